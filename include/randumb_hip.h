@@ -248,6 +248,11 @@ int rdb_linear_bwd_dcoef(float *dcoef, float *d_scale_bias, const void *dy, int6
 /* Bytes of the projection state for `desc`, or 0 when the projected form does not apply to it. */
 int64_t rdb_linear_projection_bytes(const rdb_linear_desc *desc);
 
+/* Whether a training step of the layer should keep the projection state: 1 when the projected form applies, the factored
+ * products beat the kernels that form the weight on chip (bf16: k * (in_f + out_f) < 16 * in_f * out_f), the state is at most twice
+ * the bytes of x, and the layer is not in a few-token regime, whose kernels have no projected form. */
+int rdb_linear_projection_preferred(const rdb_linear_desc *desc);
+
 /* One launch addresses at most 2^29 elements of x, y, dy or dx.  The projected entry points take any number of tokens all
  * the same: tokens are independent in y and dx and additive in dcoef, so a layer with more is run in chunks of tokens (a
  * multiple of 256 each), every chunk with a projection state of its own, one after the other in the state buffer; dcoef is

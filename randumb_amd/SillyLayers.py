@@ -165,13 +165,16 @@ class SillyLinear(SillyModuleMixin, nn.Module):
     def forward(self, input: torch.Tensor) -> torch.Tensor:
         if not self.fused:
             return F.linear(input, self.weight, self.bias)
-        w = self.weight
-        x2 = input.reshape(-1, self.in_features)
+        in_f, out_f = self.in_features, self.out_features
+        w = self._buffers["weight"]   # past nn.Module's attribute search: a few-token layer's kernels take less than a forward's host time
+        flat = input.dim() == 2
+        x2 = input if flat else input.reshape(-1, in_f)
         if x2.dtype != w.dtype:
             x2 = x2.to(w.dtype)
         sb = w.scale_bias if w.fused_bias else None
-        y = ops.linear(x2, self.weight_coef, self.in_features, self.out_features, self.in_features, 1, w.seed, sb, self.bias)
-        return y.reshape(*input.shape[:-1], self.out_features)
+        bias = self._buffers["bias"] if "bias" in self._buffers else None
+        y = ops.linear(x2, self._parameters["weight_coef"], in_f, out_f, in_f, 1, w.seed, sb, bias)
+        return y if flat else y.reshape(*input.shape[:-1], out_f)
 
     def extra_repr(self) -> str:
         return (f"in_features={self.in_features}, out_features={self.out_features}, int_dim={self.int_dim}, seeds={self.seed}, "

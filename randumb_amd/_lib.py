@@ -42,6 +42,7 @@ EXPORTS = [
     "rdb_linear_rbias_bwd",
     "rdb_linear_bwd_dcoef",
     "rdb_linear_projection_bytes",
+    "rdb_linear_projection_preferred",
     "rdb_linear_projection_chunks",
     "rdb_linear_projection_layout",
     "rdb_linear_project",
@@ -85,6 +86,24 @@ class RandumbHipError(RuntimeError):
 
 
 _lib = None
+_ext = None
+
+
+def extension():
+    """The extension module that issues a layer's calls without Python in between (``csrc/rdb_torch.cpp``), loaded once behind
+    the library it calls; raises if it has not been built."""
+    global _ext
+    if _ext is None:
+        load()
+        try:
+            from . import _rdb_torch
+        except ImportError as e:
+            raise RandumbHipError(f"randumb_amd/_rdb_torch.so cannot be loaded ({e}): build it with `make -C randumb_amd/csrc`") from e
+        from . import hip
+
+        _rdb_torch.set_hooks(RandumbHipError, hip._tick_calls)
+        _ext = _rdb_torch
+    return _ext
 
 
 def load() -> ctypes.CDLL:
@@ -137,6 +156,8 @@ def load() -> ctypes.CDLL:
     L.rdb_linear_rbias_bwd.argtypes = [vp, i64, vp, vp, i64, vp, i64, vp, dp, vp, i64, vp]
     L.rdb_linear_projection_bytes.argtypes = [dp]
     L.rdb_linear_projection_bytes.restype = i64
+    L.rdb_linear_projection_preferred.argtypes = [dp]
+    L.rdb_linear_projection_preferred.restype = ci
     L.rdb_linear_projection_chunks.argtypes = [dp, ctypes.POINTER(i64)]
     L.rdb_linear_projection_chunks.restype = ci
     L.rdb_linear_projection_layout.argtypes = [dp, ctypes.POINTER(i64)]

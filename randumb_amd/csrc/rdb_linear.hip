@@ -935,6 +935,20 @@ extern "C" int64_t rdb_linear_projection_bytes(const rdb_linear_desc *d)
     return pl.nchunks * pl.state_stride;
 }
 
+// What a training step should do with the layer: the rule behind the header's description, in integers.
+extern "C" int rdb_linear_projection_preferred(const rdb_linear_desc *d)
+{
+    if (!d || rdb_linear_projection_bytes(d) <= 0) return 0;
+    const int64_t k = d->k, in_f = d->in_f, out_f = d->out_f, T = d->tokens;
+    const bool f32 = d->act_dtype == RDB_F32;
+    // the few-token regimes, whose vector-ALU kernels have no projected form: the three one-call entry points take them
+    const bool few = k * (in_f + out_f) < in_f * out_f &&
+                     ((f32 && k <= 64 && T <= 1024) || (k <= 256 && T <= 96 && (k <= 64 || f32 || std::max(in_f, out_f) >= 1536)));
+    if (few) return 0;
+    if (f32) return k <= 2 * in_f && (k > 64 || T > 1024);   // the state holds 4 k bytes a token where x has 4 in_f: at most twice x
+    return k * (in_f + out_f) < 16 * in_f * out_f && cdiv(k, 64) * 64 <= in_f;   // 4 k bytes (k rounded up to 64) against 2 in_f
+}
+
 extern "C" int rdb_linear_projection_layout(const rdb_linear_desc *d, int64_t *info)
 {
     if (f32_projected(d)) {   // z row-major in fp32 behind the header: info[1] = 0

@@ -1,0 +1,492 @@
+// The eager path of ops.linear without Python in it: autograd functions over the C ABI of librandumb_hip.so, as the extension
+// module randumb_amd._rdb_torch.
+//
+// Why it exists: a layer's forward and backward are three to eight kernel launches of 5 to 40 us.  Issued from Python (an
+// autograd.Function, ctypes with a dozen arguments a call, a torch.empty per output, device and stream look-ups) they cost 60
+// to 75 us of host time, more than the kernels of a headline layer take (8192 tokens x 768 -> 3072, k = 256: 76 us of kernels,
+// 130 us of wall time) and twice what a single-token forward takes.  Nothing here computes: it sizes and allocates outputs
+// and workspaces with torch's allocator and calls the library.  Under torch.compile ops.linear takes the registered operators.
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <atomic>
+#include <optional>
+
+#include "../../include/randumb_hip.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+using torch::autograd::variable_list;
+
+PyObject *g_error_class = nullptr;   // randumb_amd._lib.RandumbHipError
+PyObject *g_tick = nullptr;          // hip's look at the give-up counter: called with (device index, calls)
+
+// ----------------------------------------------------------------------------------------------- errors, device, stream
+// A Python exception of the package's class, from whatever thread (the backward pass runs on autograd's).
+[[noreturn]] void fail(PyObject *cls, const std::string &msg)
+{
+    pybind11::gil_scoped_acquire gil;
+    PyErr_SetString(cls, msg.c_str());
+    python_error err;
+    err.persist();
+    throw std::move(err);
+}
+void check(int rc, const char *what)
+{
+    if (rc == 0) return;
+    fail(g_error_class ? g_error_class : PyExc_RuntimeError,
+         std::string(what) + ": " + (rc < 0 ? "argument error " : "HIP error ") + std::to_string(rc) + ": " + rdb_last_error_string());
+}
+
+void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+
+// Entry points that may run a kernel whose blocks wait for each other are counted; every 16 of them hip looks at the
+// counter of waits that gave up (which raises if there are new ones).
+void tick(const Tensor &t)
+{
+    constexpr unsigned every = 16;
+    static std::atomic<unsigned> calls[64];
+    const int dev = t.get_device();
+    if ((calls[dev & 63].fetch_add(1, std::memory_order_relaxed) + 1) % every || !g_tick) return;
+    pybind11::gil_scoped_acquire gil;
+    PyObject *r = PyObject_CallFunction(g_tick, "iI", dev, every);
+    if (!r) {
+        python_error err;
+        err.persist();
+        throw std::move(err);
+    }
+    Py_DECREF(r);
+}
+
+// ----------------------------------------------------------------------------------------------- tensors as the library reads them
+bool readable(at::ScalarType t) { return t == at::kFloat || t == at::kBFloat16; }
+int code(at::ScalarType t) { return t == at::kBFloat16 ? RDB_BF16 : RDB_F32; }
+
+Tensor native(const Tensor &t) { return (readable(t.scalar_type()) ? t : t.to(at::kFloat)).contiguous(); }
+
+// 2-D activation with unit inner stride in a dtype the kernels compute in
+Tensor act(const Tensor &t0)
+{
+    if (t0.dim() != 2) fail(PyExc_ValueError, "activations must be 2-D (tokens, features)");
+    const Tensor t = readable(t0.scalar_type()) ? t0 : t0.to(at::kFloat);
+    return t.stride(1) == 1 && t.stride(0) >= t.size(1) ? t : t.contiguous();
+}
+
+Tensor bytes(int64_t n, const Tensor &like) { return n > 0 ? at::empty({n}, like.options().dtype(at::kByte)) : Tensor(); }
+void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+struct Layer {
+    int64_t in_f, out_f, sO, sI;
+    uint32_t seed;
+};
+
+rdb_linear_desc desc(int64_t tokens, const Layer &l, int64_t k, int64_t coef_rows, at::ScalarType a, at::ScalarType c)
+{
+    rdb_linear_desc d;
+    d.tokens = tokens;
+    d.in_f = l.in_f;
+    d.out_f = l.out_f;
+    d.k = k;
+    d.coef_rows = coef_rows;
+    d.sO = l.sO;
+    d.sI = l.sI;
+    d.seed = l.seed;
+    d.act_dtype = code(a);
+    d.coef_dtype = code(c);
+    d.algo = RDB_ALGO_AUTO;
+    return d;
+}
+rdb_linear_desc desc(const Tensor &rows, const Layer &l, const Tensor &c)
+{
+    return desc(rows.size(0), l, c.size(-1), c.dim() == 1 ? 0 : c.size(0), rows.scalar_type(), c.scalar_type());
+}
+
+// ----------------------------------------------------------------------------------------------- the library's calls
+Tensor linear_fwd(const Tensor &x0, const Tensor &coefs, const Layer &l, const OptTensor &scale_bias, const OptTensor &bias)
+{
+    const Tensor x = act(x0), c = native(coefs);
+    const Tensor sb = scale_bias ? native(*scale_bias).to(c.scalar_type()) : Tensor();
+    const Tensor b = bias ? bias->to(x.scalar_type()).contiguous() : Tensor();
+    const c10::OptionalDeviceGuard guard(x.device());
+    Tensor y = at::empty({x.size(0), l.out_f}, x.options());
+    const rdb_linear_desc d = desc(x, l, c);
+    const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_FWD, &d);
+    const Tensor ws = bytes(need, x);
+    check(rdb_linear_fwd(y.data_ptr(), y.stride(0), x.data_ptr(), x.stride(0), c.data_ptr(), ptr(sb), ptr(b), &d, ptr(ws), need, stream_of(x)),
+          "rdb_linear_fwd");
+    tick(x);
+    return y;
+}
+
+Tensor linear_bwd_dx(const Tensor &dy0, const Tensor &coefs, const Layer &l, const Tensor &scale_bias)
+{
+    const Tensor dy = act(dy0), c = native(coefs);
+    const Tensor sb = scale_bias.defined() ? native(scale_bias).to(c.scalar_type()) : Tensor();
+    const c10::OptionalDeviceGuard guard(dy.device());
+    Tensor dx = at::empty({dy.size(0), l.in_f}, dy.options());
+    const rdb_linear_desc d = desc(dy, l, c);
+    const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_DX, &d);
+    const Tensor ws = bytes(need, dy);
+    check(rdb_linear_bwd_dx(dx.data_ptr(), dx.stride(0), dy.data_ptr(), dy.stride(0), c.data_ptr(), ptr(sb), &d, ptr(ws), need, stream_of(dy)),
+          "rdb_linear_bwd_dx");
+    tick(dy);
+    return dx;
+}
+
+// (dx, gradient of the random bias's scale) from one pass over the random-bias product; undefined where the library has no such kernel
+std::pair<Tensor, Tensor> linear_bwd_dx_dscale(const Tensor &dy0, const Tensor &x0, const Tensor &coefs, const Layer &l, const Tensor &scale_bias)
+{
+    if (dy0.scalar_type() != at::kBFloat16 || coefs.scalar_type() != at::kBFloat16 || coefs.dim() != 2) return {};
+    const Tensor dy = act(dy0), x = act(x0).to(dy.scalar_type()), c = native(coefs), sb = native(scale_bias).to(c.scalar_type());
+    const c10::OptionalDeviceGuard guard(dy.device());
+    const rdb_linear_desc d = desc(dy, l, c);
+    const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_DX_DSCALE, &d);
+    if (need <= 0) return {};
+    Tensor dx = at::empty({dy.size(0), l.in_f}, dy.options()), ds = at::empty({1}, dy.options().dtype(at::kFloat));
+    const Tensor ws = bytes(need, dy);
+    const int rc = rdb_linear_bwd_dx_dscale(dx.data_ptr(), dx.stride(0), ds.data_ptr<float>(), dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0),
+                                            c.data_ptr(), sb.data_ptr(), &d, ptr(ws), need, stream_of(dy));
+    if (rc == RDB_E_UNSUPPORTED) return {};   // nothing was launched
+    check(rc, "rdb_linear_bwd_dx_dscale");
+    return {dx, ds};
+}
+
+std::pair<Tensor, Tensor> linear_bwd_dcoef(const Tensor &dy0, const Tensor &x0, const Tensor &coefs, const Layer &l, bool want_scale)
+{
+    const Tensor dy = act(dy0), x = act(x0).to(dy.scalar_type());
+    const int64_t k = coefs.size(-1), rows = coefs.dim() == 1 ? 0 : coefs.size(0);
+    const c10::OptionalDeviceGuard guard(dy.device());
+    const auto f32 = dy.options().dtype(at::kFloat);
+    Tensor dc = rows ? at::empty({rows, k}, f32) : at::empty({k}, f32), ds = want_scale ? at::empty({1}, f32) : Tensor();
+    const rdb_linear_desc d = desc(dy.size(0), l, k, rows, dy.scalar_type(), at::kFloat);
+    const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_DCOEF, &d);
+    const Tensor ws = bytes(need, dy);
+    check(rdb_linear_bwd_dcoef(dc.data_ptr<float>(), want_scale ? ds.data_ptr<float>() : nullptr, dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0),
+                               &d, ptr(ws), need, stream_of(dy)),
+          "rdb_linear_bwd_dcoef");
+    return {dc, ds};
+}
+
+rdb_linear_desc rbias_desc(const Tensor &rows, const Layer &l) { return desc(rows.size(0), l, 8, l.out_f, at::kBFloat16, at::kBFloat16); }
+
+// dbias: the column sums of dy
+Tensor bias_grad(const Tensor &dy, at::ScalarType dtype) { return dy.sum(0).to(dtype); }
+
+// ----------------------------------------------------------------------------------------------- one-call form
+// y = x.W^T (+ bias) with x saved; the three products of the layer as three calls.
+class OneCallLinear : public Function<OneCallLinear> {
+  public:
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &coefs, const OptTensor &scale_bias, const OptTensor &bias, const Layer &l)
+    {
+        ctx->save_for_backward({x, coefs, scale_bias.value_or(Tensor())});
+        ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, l.sO, l.sI, (int64_t)l.seed, scale_bias ? 1 : 0,
+                                                        bias ? (int64_t)bias->scalar_type() : -1};
+        return linear_fwd(x, coefs, l, scale_bias, bias);
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &coefs = saved[1], &sb = saved[2];
+        const auto m = ctx->saved_data["layer"].toIntVector();
+        const Layer l{m[0], m[1], m[2], m[3], (uint32_t)m[4]};
+        const bool has_sb = m[5] != 0, has_bias = m[6] >= 0;
+        const at::AutoGradMode no_grad(false);
+        const bool want_dx = ctx->needs_input_grad(0), want_dc = ctx->needs_input_grad(1);
+        bool want_sb = has_sb && ctx->needs_input_grad(2);
+        const bool want_b = has_bias && ctx->needs_input_grad(has_sb ? 3 : 2);
+        const Tensor dy = grads[0].contiguous();
+        Tensor dx, dc, dsb, db;
+        if (want_dx && want_sb && l.sO == l.in_f && l.sI == 1) {
+            // the random-bias product dy.R that dx needs anyway also gives the gradient of the bias's scale (reduced against x
+            // in the same pass), so the coefficient gradient below comes from the factored kernels and dW is never formed
+            auto both = linear_bwd_dx_dscale(dy, x, coefs, l, sb);
+            if (both.first.defined()) {
+                dx = both.first;
+                dsb = both.second.to(sb.scalar_type());
+                want_sb = false;
+            }
+        }
+        if (want_dx && !dx.defined()) dx = linear_bwd_dx(dy, coefs, l, sb);
+        if (want_dc || want_sb) {
+            auto both = linear_bwd_dcoef(dy, x, coefs, l, want_sb);
+            dc = both.first.to(coefs.scalar_type());
+            if (want_sb) dsb = both.second.to(sb.scalar_type());
+        }
+        if (want_b) db = bias_grad(dy, (at::ScalarType)m[6]);
+        return {dx, dc, dsb, db, Tensor()};
+    }
+};
+
+// ----------------------------------------------------------------------------------------------- projected form
+// The forward pass keeps z = x.N^T (and, in bf16, the transposed coefficients) for the backward pass, which needs nothing else
+// of x; with the fused random bias its full-rank share is added on top in both directions and x is saved as well.
+class ProjectedLinear : public Function<ProjectedLinear> {
+  public:
+    static Tensor forward(AutogradContext *ctx, const Tensor &x0, const Tensor &coefs, const OptTensor &bias, const OptTensor &scale_bias, const Layer &l)
+    {
+        const Tensor x = act(x0), c = coefs.contiguous();
+        const c10::OptionalDeviceGuard guard(x.device());
+        const rdb_linear_desc d = desc(x, l, c);
+        const int64_t need = rdb_linear_projection_bytes(&d);
+        Tensor state = bytes(need, x), y = at::empty({x.size(0), l.out_f}, x.options());
+        const Tensor b = bias ? bias->to(x.scalar_type()).contiguous() : Tensor();
+        void *s = stream_of(x);
+        check(rdb_linear_project_fwd(y.data_ptr(), l.out_f, ptr(state), x.data_ptr(), x.stride(0), c.data_ptr(), ptr(b), &d, s), "rdb_linear_project_fwd");
+        if (scale_bias) {
+            const Tensor sb = native(*scale_bias).to(at::kBFloat16);
+            const rdb_linear_desc r = rbias_desc(x, l);
+            check(rdb_linear_rbias_fwd(y.data_ptr(), l.out_f, x.data_ptr(), x.stride(0), sb.data_ptr(), &r, s), "rdb_linear_rbias_fwd");
+        }
+        tick(x);
+        ctx->save_for_backward({state, coefs, scale_bias.value_or(Tensor()), scale_bias ? x0 : Tensor()});
+        ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, (int64_t)l.seed, scale_bias ? 1 : 0, bias ? (int64_t)bias->scalar_type() : -1};
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &state = saved[0], &coefs = saved[1], &scale_bias = saved[2];
+        const auto m = ctx->saved_data["layer"].toIntVector();
+        const Layer l{m[0], m[1], m[0], 1, (uint32_t)m[2]};
+        const bool has_sb = m[3] != 0, has_bias = m[4] >= 0;
+        const at::AutoGradMode no_grad(false);
+        const bool want_x = ctx->needs_input_grad(0), want_dc = ctx->needs_input_grad(1);
+        const bool want_b = has_bias && ctx->needs_input_grad(2), want_sb = has_sb && ctx->needs_input_grad(has_bias ? 3 : 2);
+        const bool want_dx = want_x || want_sb;   // the gradient of the scale comes out of the random-bias share of dx
+        Tensor dy = act(grads[0]);
+        const bool f32 = coefs.scalar_type() == at::kFloat;
+        if (!f32 && (dy.stride(0) % 8 || (uintptr_t)dy.data_ptr() % 16)) dy = dy.contiguous();   // rows with a leading dimension are read in place
+        const Tensor c = coefs.contiguous();
+        const c10::OptionalDeviceGuard guard(dy.device());
+        const rdb_linear_desc d = desc(dy, l, c);
+        void *s = stream_of(dy);
+        Tensor dx, dc, dsb, db;
+        if (want_dc && (want_dx || f32)) {
+            // bf16 coefficients: their gradient leaves the kernel that adds it up in bf16, where the layer runs as one chunk of tokens
+            const bool to_bf16 = !f32 && rdb_linear_projection_chunks(&d, nullptr) == 1;
+            const int64_t need = rdb_linear_workspace_bytes(to_bf16 ? RDB_OP_LINEAR_BWD_PROJECTED_TO : RDB_OP_LINEAR_BWD_PROJECTED, &d);
+            const Tensor ws = bytes(need, dy);
+            if (want_dx) dx = at::empty({dy.size(0), l.in_f}, dy.options());
+            dc = at::empty({c.size(0), c.size(1)}, dy.options().dtype(to_bf16 ? at::kBFloat16 : at::kFloat));
+            check(to_bf16 ? rdb_linear_bwd_projected_to(ptr(dx), l.in_f, dc.data_ptr(), RDB_BF16, dy.data_ptr(), dy.stride(0), state.data_ptr(), c.data_ptr(),
+                                                        &d, ptr(ws), need, s)
+                          : rdb_linear_bwd_projected(ptr(dx), l.in_f, dc.data_ptr<float>(), dy.data_ptr(), dy.stride(0), state.data_ptr(), c.data_ptr(), &d,
+                                                     ptr(ws), need, s),
+                  "rdb_linear_bwd_projected");
+            dc = dc.to(c.scalar_type());
+        } else if (want_dx) {
+            dx = linear_bwd_dx(dy, c, l, Tensor());
+        } else if (want_dc) {
+            dc = at::empty({c.size(0), c.size(1)}, dy.options().dtype(at::kFloat));
+            check(rdb_linear_bwd_dcoef_projected(dc.data_ptr<float>(), dy.data_ptr(), dy.stride(0), state.data_ptr(), &d, s), "rdb_linear_bwd_dcoef_projected");
+            dc = dc.to(c.scalar_type());
+        }
+        if (has_sb && dx.defined()) {
+            const Tensor x = act(saved[3]), sb = native(scale_bias).to(at::kBFloat16);
+            const rdb_linear_desc r = rbias_desc(dy, l);
+            if (want_sb) {
+                const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_BWD, &r);
+                const Tensor ws = bytes(need, dy);
+                dsb = at::empty({1}, dy.options().dtype(at::kFloat));
+                check(rdb_linear_rbias_bwd(dx.data_ptr(), l.in_f, dsb.data_ptr<float>(), dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), sb.data_ptr(),
+                                           &r, ptr(ws), need, s),
+                      "rdb_linear_rbias_bwd");
+                dsb = dsb.to(scale_bias.scalar_type());
+            } else {
+                check(rdb_linear_rbias_bwd(dx.data_ptr(), l.in_f, nullptr, dy.data_ptr(), dy.stride(0), nullptr, 0, sb.data_ptr(), &r, nullptr, 0, s),
+                      "rdb_linear_rbias_bwd");
+            }
+        }
+        if (!want_x) dx = Tensor();
+        if (want_b) db = bias_grad(dy, (at::ScalarType)m[4]);
+        return {dx, dc, db, dsb, Tensor()};
+    }
+};
+
+// ----------------------------------------------------------------------------------------------- a pseudorandom vector (a layer's bias)
+// b[o] = sum_m noise(PRIME*o + m) coef[m] (+ s noise1d(o)), in the coefficients' dtype, and the gradients of coef and s.
+class VectorFromCoefs : public Function<VectorFromCoefs> {
+  public:
+    static Tensor forward(AutogradContext *ctx, const Tensor &coef, const OptTensor &scale_bias, int64_t n, int64_t seed)
+    {
+        ctx->saved_data["vector"] = std::vector<int64_t>{coef.numel(), seed, (int64_t)coef.scalar_type(), scale_bias ? (int64_t)scale_bias->scalar_type() : -1};
+        return values(coef, scale_bias, n, seed);
+    }
+    static Tensor values(const Tensor &coef, const OptTensor &scale_bias, int64_t n, int64_t seed)
+    {
+        const Tensor c = native(coef), sb = scale_bias ? native(*scale_bias).to(c.scalar_type()) : Tensor();
+        const c10::OptionalDeviceGuard guard(c.device());
+        Tensor out = at::empty({n}, c.options().dtype(at::kFloat));
+        check(rdb_materialize_fwd(out.data_ptr<float>(), c.data_ptr(), code(c.scalar_type()), 0, c.numel(), 0, 1, n, 0, 1, (uint32_t)seed, ptr(sb), stream_of(c)),
+              "rdb_materialize_fwd");
+        return out.to(coef.scalar_type());
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const auto m = ctx->saved_data["vector"].toIntVector();
+        const at::AutoGradMode no_grad(false);
+        const Tensor d = native(grads[0]);
+        const c10::OptionalDeviceGuard guard(d.device());
+        const auto f32 = d.options().dtype(at::kFloat);
+        Tensor dc, ds;
+        if (ctx->needs_input_grad(0)) {
+            const int64_t need = rdb_materialize_bwd_workspace_bytes(0, m[0], 0, d.numel());
+            const Tensor ws = bytes(need, d);
+            dc = at::empty({m[0]}, f32);
+            check(rdb_materialize_bwd(dc.data_ptr<float>(), d.data_ptr(), code(d.scalar_type()), 0, m[0], 0, d.numel(), (uint32_t)m[1], ptr(ws), need,
+                                      stream_of(d)),
+                  "rdb_materialize_bwd");
+            dc = dc.to((at::ScalarType)m[2]);
+        }
+        if (m[3] >= 0 && ctx->needs_input_grad(1)) {
+            const int64_t need = rdb_scale_bias_bwd_workspace_bytes(d.numel());
+            const Tensor ws = bytes(need, d);
+            ds = at::empty({1}, f32);
+            check(rdb_scale_bias_bwd(ds.data_ptr<float>(), d.data_ptr(), code(d.scalar_type()), d.numel(), (uint32_t)m[1], ptr(ws), need, stream_of(d)),
+                  "rdb_scale_bias_bwd");
+            ds = ds.to((at::ScalarType)m[3]);
+        }
+        return {dc, ds, Tensor(), Tensor()};
+    }
+};
+
+// ----------------------------------------------------------------------------------------------- Python methods
+struct BadArgument {};
+
+const Tensor &tensor_arg(PyObject *o)
+{
+    if (!THPVariable_Check(o)) {
+        PyErr_SetString(PyExc_TypeError, "expected a tensor");
+        throw BadArgument();
+    }
+    return THPVariable_Unpack(o);
+}
+OptTensor opt_arg(PyObject *o) { return o == Py_None ? OptTensor() : OptTensor(tensor_arg(o)); }
+int64_t int_arg(PyObject *o)
+{
+    const long long v = PyLong_AsLongLong(o);
+    if (v == -1 && PyErr_Occurred()) throw BadArgument();
+    return v;
+}
+uint32_t seed_arg(PyObject *o)
+{
+    const int64_t v = int_arg(o);
+    if (v < 0 || v >= (1ll << 32)) {
+        PyErr_Format(PyExc_ValueError, "seed must fit in 32 unsigned bits, got %lld", (long long)v);
+        throw BadArgument();
+    }
+    return (uint32_t)v;
+}
+void count_args(Py_ssize_t n, Py_ssize_t want)
+{
+    if (n == want) return;
+    PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", want, n);
+    throw BadArgument();
+}
+bool wants_grad(const OptTensor &t) { return t && t->requires_grad(); }
+
+template <typename F> PyObject *guarded(F f)
+{
+    try {
+        return f();
+    } catch (const BadArgument &) {
+        return nullptr;
+    } catch (python_error &e) {
+        e.restore();
+        return nullptr;
+    } catch (const std::exception &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return nullptr;
+    }
+}
+
+// takes_projected(x, coefs, in_f, out_f, sO, sI, scale_bias, bias): whether ops.linear runs the projected form
+PyObject *py_takes_projected(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 8);
+        const Tensor &x = tensor_arg(a[0]), &c = tensor_arg(a[1]);
+        const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[4]), int_arg(a[5]), 0};
+        bool yes = c.dim() == 2 && c.size(0) == l.out_f && l.sO == l.in_f && l.sI == 1 && x.is_cuda() && x.dim() == 2 && readable(x.scalar_type()) &&
+                   c.scalar_type() == x.scalar_type();
+        if (yes && a[6] != Py_None) yes = x.scalar_type() == at::kBFloat16 && l.in_f % 8 == 0 && l.out_f % 8 == 0 && tensor_arg(a[6]).numel() == 1;
+        if (yes && a[7] != Py_None) yes = tensor_arg(a[7]).scalar_type() == x.scalar_type();
+        if (yes) {
+            const rdb_linear_desc d = desc(x, l, c);
+            yes = rdb_linear_projection_preferred(&d) != 0;
+        }
+        return PyBool_FromLong(yes);
+    });
+}
+
+// linear_projected(x, coefs, in_f, out_f, seed, bias, scale_bias)
+PyObject *py_linear_projected(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 7);
+        const Tensor &x = tensor_arg(a[0]), &c = tensor_arg(a[1]);
+        const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[2]), 1, seed_arg(a[4])};
+        const OptTensor bias = opt_arg(a[5]), sb = opt_arg(a[6]);
+        // without a backward pass to come there is no state to keep: the one-call forward
+        if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(bias) || wants_grad(sb)))
+            return THPVariable_Wrap(linear_fwd(x, c, l, sb, bias));
+        return THPVariable_Wrap(ProjectedLinear::apply(x, c, bias, sb, l));
+    });
+}
+
+// linear_one_call(x, coefs, in_f, out_f, sO, sI, seed, scale_bias, bias)
+PyObject *py_linear_one_call(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 9);
+        const Tensor &x = tensor_arg(a[0]), &c = tensor_arg(a[1]);
+        const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[4]), int_arg(a[5]), seed_arg(a[6])};
+        const OptTensor sb = opt_arg(a[7]), bias = opt_arg(a[8]);
+        if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(bias) || wants_grad(sb)))
+            return THPVariable_Wrap(linear_fwd(x, c, l, sb, bias));
+        return THPVariable_Wrap(OneCallLinear::apply(x, c, sb, bias, l));
+    });
+}
+
+// vector_from_coefs(coef, scale_bias, n, seed): a contiguous vector-coef tensor of n elements, differentiable in coef and scale_bias
+PyObject *py_vector_from_coefs(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 4);
+        const Tensor &c = tensor_arg(a[0]);
+        const OptTensor sb = opt_arg(a[1]);
+        const int64_t len = int_arg(a[2]), seed = seed_arg(a[3]);
+        if (!at::GradMode::is_enabled() || !(c.requires_grad() || wants_grad(sb))) return THPVariable_Wrap(VectorFromCoefs::values(c, sb, len, seed));
+        return THPVariable_Wrap(VectorFromCoefs::apply(c, sb, len, seed));
+    });
+}
+
+// set_hooks(error class, tick)
+PyObject *py_set_hooks(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 2);
+        Py_INCREF(a[0]);
+        Py_INCREF(a[1]);
+        Py_XSETREF(g_error_class, a[0]);
+        Py_XSETREF(g_tick, a[1]);
+        Py_RETURN_NONE;
+    });
+}
+
+#define RDB_METHOD(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {RDB_METHOD(takes_projected),   RDB_METHOD(linear_projected), RDB_METHOD(linear_one_call),
+                         RDB_METHOD(vector_from_coefs), RDB_METHOD(set_hooks),        {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_rdb_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__rdb_torch(void) { return PyModule_Create(&module); }

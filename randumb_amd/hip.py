@@ -114,12 +114,13 @@ class SyncWatch:
                 "for were filled with NaN, and projection states and recorded graphs of those launches must not be used again. "
                 "The library now runs producers and consumers as separate launches (rdb_set_one_launch(0)).")
 
-    def tick(self, stream) -> None:
-        """Called by the entry points that may run a one-launch kernel; never waits for the device."""
-        self.calls += 1
+    def tick(self, stream, calls: int = 1) -> None:
+        """Called by the entry points that may run a one-launch kernel (or once per several of their calls); never waits for the
+        device."""
+        before, self.calls = self.calls, self.calls + calls
         if self.pending is not None and self.pending.query():
             self._judge()
-        if self.pending is None and self.calls % self.every == 0:
+        if self.pending is None and before // self.every != self.calls // self.every:
             self._enqueue(stream)
 
     def check(self, stream) -> None:
@@ -139,6 +140,12 @@ def _watch(device) -> SyncWatch:
     if w is None:
         w = _watches[key] = SyncWatch()
     return w
+
+
+def _tick_calls(index: int, calls: int) -> None:
+    """What the extension module calls after every ``calls`` of its calls on device ``index``."""
+    dev = torch.device("cuda", index)
+    _watch(dev).tick(_stream(dev), calls)
 
 
 def sync_check(device="cuda") -> None:

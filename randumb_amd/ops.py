@@ -18,7 +18,7 @@ import torch
 from torch import Tensor
 from torch.library import custom_op
 
-from . import hip
+from . import _lib, hip
 
 __all__ = [
     "materialize_fwd", "materialize_bwd", "scale_bias_bwd", "embed_fwd", "embed_bwd",
@@ -273,8 +273,9 @@ def _dense(t: Optional[Tensor]) -> Optional[Tensor]:
     return t.get_materialized() if t is not None and hasattr(t, "get_materialized") else t
 
 
-class _EagerLinear(torch.autograd.Function):
-    """``rten::linear_fwd`` and its registered backward, without the operator wrappers: what ``linear`` runs eagerly."""
+class _OneCallFunction(torch.autograd.Function):
+    """``rten::linear_fwd`` and its registered backward in Python, without the operator wrappers: for the few requests the
+    extension module does not take (a bias that is a pseudorandom tensor of another form than a layer's)."""
 
     @staticmethod
     def forward(ctx, x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias):
@@ -309,7 +310,7 @@ class _EagerLinear(torch.autograd.Function):
         return dx, dcoefs, None, None, None, None, None, dsb, dbias
 
 
-class _ProjectedLinear(torch.autograd.Function):
+class _ProjectedFunction(torch.autograd.Function):
     """``y = x @ W.T (+ bias)`` for a matrix-coef weight in bf16 or fp32.  The forward pass computes the projection state
     (``z = x @ Noise.T`` in the element orders its consumers read, and for bf16 the transposed coefficients) once and saves it
     for the backward pass, which then needs nothing else of ``x``; the reference's autograd saves ``x`` and materialises ``W``
@@ -372,11 +373,43 @@ class _ProjectedLinear(torch.autograd.Function):
         return dx, dcoefs, None, None, None, dbias, dsb
 
 
+def _rbias_dense(t) -> Optional[Tensor]:
+    """A layer's pseudorandom bias as a dense tensor with autograd behind it (its coefficients and scale), or None where the
+    tensor is not a contiguous vector-coef one in its coefficients' dtype."""
+    if t.coef_rows or t.dim() != 1 or t.stride(0) != 1 or t.dtype != t._coef.dtype or type(t._coef) not in (Tensor, torch.nn.Parameter):
+        return None
+    c, sb = t._coef, t.scale_bias if t.fused_bias else None
+    if not t.requires_grad:
+        c, sb = c.detach(), None if sb is None else sb.detach()
+    return _lib.extension().vector_from_coefs(c, sb, t.shape[0], t.seed)
+
+
+class _ProjectedLinear:
+    """The projected form as ``linear`` runs it: eagerly by the extension module, whose autograd function is
+    :class:`_ProjectedFunction` in C++; under torch.compile (and when the state's copy of the coefficients is to be checked) that one."""
+
+    @staticmethod
+    def apply(x, coefs, in_features, out_features, seed, bias, scale_bias=None):
+        if _tracing() or hip.CHECK_STATE_COEF or hasattr(bias, "get_materialized"):
+            return _ProjectedFunction.apply(x, coefs, in_features, out_features, seed, bias, scale_bias)
+        return _lib.extension().linear_projected(x, coefs, in_features, out_features, seed, bias, scale_bias)
+
+
 def linear(x: Tensor, coefs: Tensor, in_features: int, out_features: int, stride_o: int, stride_i: int, seed: int,
            scale_bias: Optional[Tensor], bias: Optional[Tensor]) -> Tensor:
     """``x @ W.T (+ bias)`` with autograd, choosing the projected form when the layer qualifies (matrix-coef; bf16 with sizes in
     multiples of 8, or fp32 beyond the few-token regime; the fused random bias in bf16 when run eagerly) and
     ``rten::linear_fwd`` otherwise.  Same arguments as ``rten::linear_fwd``."""
+    if x.is_cuda and not _tracing():
+        ext = _lib._ext or _lib.extension()
+        if hasattr(bias, "get_materialized"):
+            dense = _rbias_dense(bias)
+            bias = bias if dense is None else dense
+        if ext.takes_projected(x, coefs, in_features, out_features, stride_o, stride_i, scale_bias, bias):
+            return _ProjectedLinear.apply(x, coefs, in_features, out_features, seed, bias, scale_bias)
+        if hasattr(bias, "get_materialized"):
+            return _OneCallFunction.apply(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias)
+        return ext.linear_one_call(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias)
     rbias_ok = scale_bias is None or (x.dtype == torch.bfloat16 and scale_bias.numel() == 1 and not _tracing()
                                       and hip.linear_rbias_supported(in_features, out_features, x.dtype))
     if (rbias_ok and coefs.dim() == 2 and coefs.shape[0] == out_features and stride_o == in_features and stride_i == 1
@@ -384,8 +417,6 @@ def linear(x: Tensor, coefs: Tensor, in_features: int, out_features: int, stride
             and (bias is None or bias.dtype == x.dtype)
             and hip.linear_projection_preferred(x.shape[0], in_features, out_features, coefs.shape[1], x.dtype)):
         return _ProjectedLinear.apply(x, coefs, in_features, out_features, seed, bias, scale_bias)
-    if x.is_cuda and not _tracing():
-        return _EagerLinear.apply(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias)
     return linear_fwd(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias)
 
 

@@ -11,6 +11,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <atomic>
@@ -489,4 +490,18 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_rdb_torch", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__rdb_torch(void) { return PyModule_Create(&module); }
+// The name under which a function's node shows up as grad_fn in Python.
+template <typename F> static void name_node(const char *name)
+{
+    static PyTypeObject type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+    torch::autograd::_initFunctionPyTypeObject(type, name, nullptr, nullptr);
+    torch::autograd::registerCppFunction(typeid(torch::autograd::CppNode<F>), &type);
+}
+
+PyMODINIT_FUNC PyInit__rdb_torch(void)
+{
+    name_node<OneCallLinear>("OneCallLinearBackward");
+    name_node<ProjectedLinear>("ProjectedLinearBackward");
+    name_node<VectorFromCoefs>("VectorFromCoefsBackward");
+    return PyModule_Create(&module);
+}

@@ -372,6 +372,41 @@ int rdb_sync_giveups(uint32_t *count, void *stream);
 int rdb_selftest_sync_giveup(void *y, int64_t ldy, void *scratch, int64_t scratch_bytes, const void *coef,
                              const rdb_linear_desc *desc, int polls, void *stream);
 
+/* ------------------------------------------------------------------------------------------ around the linears of a block
+ * The parts of a transformer block between its pseudorandom linears, in bf16 with fp32 arithmetic, each as one pass (or one
+ * fused product) where a chain of stock operators makes several; values are rounded to bf16 at the same places as there.
+ * Replace, in modded-nanogpt/gpt_models.py: norm (22-23) and the residual addition in front of it, F.relu(x).square(),
+ * F.cross_entropy(logits.float(), target) (mean over the rows that count), Rotary (29-49) and CausalSelfAttention (201-232)
+ * with plain causal attention.  All tensors contiguous, RDB_BF16 unless stated. */
+
+/* y = x' * rstd, rstd[row] = 1 / sqrt(mean(x'^2) + eps) (fp32 [rows]) with x' = x, or x' = sum = x + delta when delta != NULL.
+ * dim a multiple of 4, at most 4096 (RDB_E_UNSUPPORTED otherwise); 8-byte aligned pointers. */
+int rdb_rms_norm_fwd(void *y, void *sum, float *rstd, const void *x, const void *delta, int64_t rows, int64_t dim, float eps, void *stream);
+/* dx of the normalisation of x, plus dsum (the gradient that reaches x + delta past it) when dsum != NULL. */
+int rdb_rms_norm_bwd(void *dx, const void *dy, const void *x, const void *dsum, const float *rstd, int64_t rows, int64_t dim, void *stream);
+
+/* dy == NULL: out = relu(x)^2;  otherwise out = dy * 2 relu(x).  n elements, 16-byte aligned pointers. */
+int rdb_relu_square(void *out, const void *x, const void *dy, int64_t n, void *stream);
+
+/* loss[0] (fp32) = mean over the rows with target != ignore_index of log(sum exp(logits[row])) - logits[row][target[row]].
+ * scratch: 2 * rows + 1 floats; its first rows + 1 are what the backward call needs.  A target outside the classes gives NaN.
+ * classes a multiple of 8, 16-byte aligned logits (RDB_E_UNSUPPORTED otherwise). */
+int rdb_cross_entropy_fwd(float *loss, float *scratch, const void *logits, const int64_t *target, int64_t rows, int64_t classes,
+                          int64_t ignore_index, void *stream);
+int rdb_cross_entropy_bwd(void *dlogits, const void *logits, const int64_t *target, const float *scratch, const float *dloss,
+                          int64_t rows, int64_t classes, int64_t ignore_index, void *stream);
+
+/* Causal self-attention, head dimension 64: qkv [batch][T][3][heads][64] -> y [batch][T][heads][64]; q and k are normalised over the
+ * head dimension (eps) and rotated by position * inv_freq[32] (dtype inv_freq_dtype; bf16 frequencies make angle, cosine and sine
+ * bf16), then y = softmax(q k^T / 8) v over the positions up to each token's own.  q, k: [batch * heads][T][64] and scratch:
+ * rdb_causal_attention_scratch_floats(...) floats, kept for the backward call, which writes all of dqkv.  A sequence's qkv
+ * must stay below 2^30 bytes (RDB_E_UNSUPPORTED otherwise); 16-byte aligned pointers. */
+int64_t rdb_causal_attention_scratch_floats(int64_t batch, int64_t T, int64_t heads);
+int rdb_causal_attention_fwd(void *y, void *q, void *k, float *scratch, const void *qkv, const void *inv_freq, int inv_freq_dtype,
+                             int64_t batch, int64_t T, int64_t heads, float eps, void *stream);
+int rdb_causal_attention_bwd(void *dqkv, const void *dy, const void *y, const void *q, const void *k, float *scratch, const void *qkv,
+                             int64_t batch, int64_t T, int64_t heads, float eps, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

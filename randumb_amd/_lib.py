@@ -58,6 +58,14 @@ EXPORTS = [
     "rdb_sync_giveups_async",
     "rdb_sync_giveups",
     "rdb_selftest_sync_giveup",
+    "rdb_rms_norm_fwd",
+    "rdb_rms_norm_bwd",
+    "rdb_relu_square",
+    "rdb_cross_entropy_fwd",
+    "rdb_cross_entropy_bwd",
+    "rdb_causal_attention_scratch_floats",
+    "rdb_causal_attention_fwd",
+    "rdb_causal_attention_bwd",
 ]
 
 ABI_VERSION = 8   # what this binding was written against (rdb_abi_version)

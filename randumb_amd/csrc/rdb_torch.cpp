@@ -359,6 +359,155 @@ class VectorFromCoefs : public Function<VectorFromCoefs> {
     }
 };
 
+// ----------------------------------------------------------------------------------------------- the rest of a transformer block
+// bf16 on the GPU; what gpt.py calls when its tensors are that.
+void need_bf16(const char *who, const Tensor &t)
+{
+    if (!t.is_cuda() || t.scalar_type() != at::kBFloat16) fail(PyExc_ValueError, std::string(who) + " needs bf16 tensors on the GPU");
+}
+int64_t row_count(const Tensor &x) { return x.size(-1) ? x.numel() / x.size(-1) : 0; }
+
+// x -> x / rms(x) over the last dimension
+class RmsNorm : public Function<RmsNorm> {
+  public:
+    static Tensor forward(AutogradContext *ctx, const Tensor &x0, double eps)
+    {
+        const Tensor x = x0.contiguous();
+        const c10::OptionalDeviceGuard guard(x.device());
+        Tensor y = at::empty_like(x), rstd = at::empty({row_count(x)}, x.options().dtype(at::kFloat));
+        check(rdb_rms_norm_fwd(y.data_ptr(), nullptr, rstd.data_ptr<float>(), x.data_ptr(), nullptr, row_count(x), x.size(-1), (float)eps, stream_of(x)),
+              "rdb_rms_norm_fwd");
+        ctx->save_for_backward({x, rstd});
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const at::AutoGradMode no_grad(false);
+        const Tensor &x = saved[0], dy = grads[0].contiguous();
+        const c10::OptionalDeviceGuard guard(x.device());
+        Tensor dx = at::empty_like(x);
+        check(rdb_rms_norm_bwd(dx.data_ptr(), dy.data_ptr(), x.data_ptr(), nullptr, saved[1].data_ptr<float>(), row_count(x), x.size(-1), stream_of(x)),
+              "rdb_rms_norm_bwd");
+        return {dx, Tensor()};
+    }
+};
+
+// (x, delta) -> (x + delta, its normalisation)
+class AddRmsNorm : public Function<AddRmsNorm> {
+  public:
+    static variable_list forward(AutogradContext *ctx, const Tensor &x0, const Tensor &delta0, double eps)
+    {
+        const Tensor x = x0.contiguous(), delta = delta0.contiguous();
+        const c10::OptionalDeviceGuard guard(x.device());
+        Tensor y = at::empty_like(x), sum = at::empty_like(x), rstd = at::empty({row_count(x)}, x.options().dtype(at::kFloat));
+        check(rdb_rms_norm_fwd(y.data_ptr(), sum.data_ptr(), rstd.data_ptr<float>(), x.data_ptr(), delta.data_ptr(), row_count(x), x.size(-1), (float)eps,
+                               stream_of(x)),
+              "rdb_rms_norm_fwd");
+        ctx->save_for_backward({sum, rstd});
+        ctx->set_materialize_grads(false);
+        return {sum, y};
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const at::AutoGradMode no_grad(false);
+        if (!grads[1].defined()) return {grads[0], grads[0], Tensor()};
+        const Tensor &x = saved[0], dy = grads[1].contiguous(), dsum = grads[0].defined() ? grads[0].contiguous() : Tensor();
+        const c10::OptionalDeviceGuard guard(x.device());
+        Tensor dx = at::empty_like(x);
+        check(rdb_rms_norm_bwd(dx.data_ptr(), dy.data_ptr(), x.data_ptr(), ptr(dsum), saved[1].data_ptr<float>(), row_count(x), x.size(-1), stream_of(x)),
+              "rdb_rms_norm_bwd");
+        return {dx, dx, Tensor()};
+    }
+};
+
+class ReluSquare : public Function<ReluSquare> {
+  public:
+    static Tensor forward(AutogradContext *ctx, const Tensor &x0)
+    {
+        const Tensor x = x0.contiguous();
+        const c10::OptionalDeviceGuard guard(x.device());
+        Tensor y = at::empty_like(x);
+        check(rdb_relu_square(y.data_ptr(), x.data_ptr(), nullptr, x.numel(), stream_of(x)), "rdb_relu_square");
+        ctx->save_for_backward({x});
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const Tensor x = ctx->get_saved_variables()[0];
+        const at::AutoGradMode no_grad(false);
+        const Tensor dy = grads[0].contiguous();
+        const c10::OptionalDeviceGuard guard(x.device());
+        Tensor dx = at::empty_like(x);
+        check(rdb_relu_square(dx.data_ptr(), x.data_ptr(), dy.data_ptr(), x.numel(), stream_of(x)), "rdb_relu_square");
+        return {dx};
+    }
+};
+
+// mean cross entropy of bf16 logits (rows, classes), computed in fp32
+class CrossEntropy : public Function<CrossEntropy> {
+  public:
+    static Tensor forward(AutogradContext *ctx, const Tensor &logits0, const Tensor &target0, int64_t ignore)
+    {
+        const Tensor logits = logits0.contiguous(), target = target0.contiguous();
+        const c10::OptionalDeviceGuard guard(logits.device());
+        const int64_t rows = logits.size(0);
+        Tensor loss = at::empty({}, logits.options().dtype(at::kFloat)), scratch = at::empty({2 * rows + 1}, loss.options());
+        check(rdb_cross_entropy_fwd(loss.data_ptr<float>(), scratch.data_ptr<float>(), logits.data_ptr(), target.data_ptr<int64_t>(), rows, logits.size(1), ignore,
+                                    stream_of(logits)),
+              "rdb_cross_entropy_fwd");
+        ctx->save_for_backward({logits, target, scratch});
+        ctx->saved_data["ignore"] = ignore;
+        return loss;
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const at::AutoGradMode no_grad(false);
+        const Tensor &logits = saved[0], dloss = grads[0].to(at::kFloat).contiguous();
+        const c10::OptionalDeviceGuard guard(logits.device());
+        Tensor d = at::empty_like(logits);
+        check(rdb_cross_entropy_bwd(d.data_ptr(), logits.data_ptr(), saved[1].data_ptr<int64_t>(), saved[2].data_ptr<float>(), dloss.data_ptr<float>(),
+                                    logits.size(0), logits.size(1), ctx->saved_data["ignore"].toInt(), stream_of(logits)),
+              "rdb_cross_entropy_bwd");
+        return {d, Tensor(), Tensor()};
+    }
+};
+
+// qkv (B, T, 3 * heads * 64) -> causal self-attention with normalised, rotated q and k (B, T, heads * 64)
+class CausalAttention : public Function<CausalAttention> {
+  public:
+    static Tensor forward(AutogradContext *ctx, const Tensor &qkv0, const Tensor &inv_freq0, int64_t heads, double eps)
+    {
+        const Tensor qkv = qkv0.contiguous(), inv_freq = native(inv_freq0);
+        const c10::OptionalDeviceGuard guard(qkv.device());
+        const int64_t B = qkv.size(0), T = qkv.size(1);
+        Tensor y = at::empty({B, T, heads * 64}, qkv.options()), q = at::empty({B * heads, T, 64}, qkv.options()), k = at::empty_like(q);
+        Tensor scratch = at::empty({rdb_causal_attention_scratch_floats(B, T, heads)}, qkv.options().dtype(at::kFloat));
+        check(rdb_causal_attention_fwd(y.data_ptr(), q.data_ptr(), k.data_ptr(), scratch.data_ptr<float>(), qkv.data_ptr(), inv_freq.data_ptr(),
+                                       code(inv_freq.scalar_type()), B, T, heads, (float)eps, stream_of(qkv)),
+              "rdb_causal_attention_fwd");
+        ctx->save_for_backward({qkv, y, q, k, scratch});
+        ctx->saved_data["heads"] = heads;
+        ctx->saved_data["eps"] = eps;
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const at::AutoGradMode no_grad(false);
+        const Tensor &qkv = saved[0], dy = grads[0].contiguous();
+        const c10::OptionalDeviceGuard guard(qkv.device());
+        Tensor d = at::empty_like(qkv);
+        check(rdb_causal_attention_bwd(d.data_ptr(), dy.data_ptr(), saved[1].data_ptr(), saved[2].data_ptr(), saved[3].data_ptr(), saved[4].data_ptr<float>(),
+                                       qkv.data_ptr(), qkv.size(0), qkv.size(1), ctx->saved_data["heads"].toInt(), (float)ctx->saved_data["eps"].toDouble(),
+                                       stream_of(qkv)),
+              "rdb_causal_attention_bwd");
+        return {d, Tensor(), Tensor(), Tensor()};
+    }
+};
+
 // ----------------------------------------------------------------------------------------------- Python methods
 struct BadArgument {};
 
@@ -470,6 +619,76 @@ PyObject *py_vector_from_coefs(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
 }
 
+double float_arg(PyObject *o)
+{
+    const double v = PyFloat_AsDouble(o);
+    if (v == -1.0 && PyErr_Occurred()) throw BadArgument();
+    return v;
+}
+
+// rms_norm(x, eps)
+PyObject *py_rms_norm(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 2);
+        const Tensor &x = tensor_arg(a[0]);
+        need_bf16("rms_norm", x);
+        return THPVariable_Wrap(RmsNorm::apply(x, float_arg(a[1])));
+    });
+}
+
+// add_rms_norm(x, delta, eps) -> (x + delta, its normalisation)
+PyObject *py_add_rms_norm(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 3);
+        const Tensor &x = tensor_arg(a[0]), &delta = tensor_arg(a[1]);
+        need_bf16("add_rms_norm", x);
+        need_bf16("add_rms_norm", delta);
+        if (x.sizes() != delta.sizes()) fail(PyExc_ValueError, "add_rms_norm needs tensors of one shape");
+        const auto r = AddRmsNorm::apply(x, delta, float_arg(a[2]));
+        PyObject *s = THPVariable_Wrap(r[0]), *y = THPVariable_Wrap(r[1]);
+        return Py_BuildValue("NN", s, y);
+    });
+}
+
+PyObject *py_relu_square(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 1);
+        const Tensor &x = tensor_arg(a[0]);
+        need_bf16("relu_square", x);
+        return THPVariable_Wrap(ReluSquare::apply(x));
+    });
+}
+
+// cross_entropy(logits, target, ignore_index): mean over the rows that count
+PyObject *py_cross_entropy(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 3);
+        const Tensor &x = tensor_arg(a[0]), &t = tensor_arg(a[1]);
+        need_bf16("cross_entropy", x);
+        if (x.dim() != 2 || t.dim() != 1 || t.size(0) != x.size(0) || t.scalar_type() != at::kLong || t.device() != x.device())
+            fail(PyExc_ValueError, "cross_entropy needs logits (rows, classes) and int64 targets (rows) on one device");
+        return THPVariable_Wrap(CrossEntropy::apply(x, t, int_arg(a[2])));
+    });
+}
+
+// causal_attention(qkv, inv_freq, heads, eps)
+PyObject *py_causal_attention(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 4);
+        const Tensor &qkv = tensor_arg(a[0]), &f = tensor_arg(a[1]);
+        const int64_t heads = int_arg(a[2]);
+        need_bf16("causal_attention", qkv);
+        if (qkv.dim() != 3 || qkv.size(2) != 3 * heads * 64 || f.numel() != 32 || f.device() != qkv.device())
+            fail(PyExc_ValueError, "causal_attention needs qkv (B, T, 3 * heads * 64) and 32 frequencies on one device");
+        return THPVariable_Wrap(CausalAttention::apply(qkv, f, heads, float_arg(a[3])));
+    });
+}
+
 // set_hooks(error class, tick)
 PyObject *py_set_hooks(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
@@ -485,7 +704,9 @@ PyObject *py_set_hooks(PyObject *, PyObject *const *a, Py_ssize_t n)
 
 #define RDB_METHOD(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {RDB_METHOD(takes_projected),   RDB_METHOD(linear_projected), RDB_METHOD(linear_one_call),
-                         RDB_METHOD(vector_from_coefs), RDB_METHOD(set_hooks),        {nullptr, nullptr, 0, nullptr}};
+                         RDB_METHOD(vector_from_coefs), RDB_METHOD(set_hooks),        RDB_METHOD(rms_norm),
+                         RDB_METHOD(add_rms_norm),      RDB_METHOD(relu_square),      RDB_METHOD(cross_entropy),
+                         RDB_METHOD(causal_attention),  {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_rdb_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
@@ -503,5 +724,10 @@ PyMODINIT_FUNC PyInit__rdb_torch(void)
     name_node<OneCallLinear>("OneCallLinearBackward");
     name_node<ProjectedLinear>("ProjectedLinearBackward");
     name_node<VectorFromCoefs>("VectorFromCoefsBackward");
+    name_node<RmsNorm>("RmsNormBackward");
+    name_node<AddRmsNorm>("AddRmsNormBackward");
+    name_node<ReluSquare>("ReluSquareBackward");
+    name_node<CrossEntropy>("CrossEntropyBackward");
+    name_node<CausalAttention>("CausalAttentionBackward");
     return PyModule_Create(&module);
 }

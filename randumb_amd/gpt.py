@@ -7,7 +7,9 @@ dimension k and seeds taken in layer order from one generator (0..47 for 12 laye
 scaled-dot-product attention (the reference's FlexAttention document mask needs a tracing compiler); the token embedding
 and the language-model head are ordinary dense layers unless the configuration asks for the reference's random-backed ones
 (modded-nanogpt/gpt_models.py:303, 310).  Everything that is not a random-backed linear is stock PyTorch: this file
-wires layers, the kernels are reached through SillyLinear.
+wires layers, the kernels are reached through SillyLinear.  In bf16 on the GPU, run eagerly, the rest of a block (normalisation,
+rotary attention with a head dimension of 64, squared ReLU, the loss) is not stock either: chains of stock operators took 6 times
+what the linears' kernels take, most of it in passes over memory that the fused ones do not make.
 """
 from dataclasses import dataclass
 from typing import Generator
@@ -16,11 +18,39 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from . import _lib
 from .SillyLayers import SillyEmbedding, SillyLinear
 
 
+def _fused(x: torch.Tensor):
+    """The extension module where ``x`` is what its kernels take, else None: bf16 on the GPU, run eagerly."""
+    if x.dtype is torch.bfloat16 and x.is_cuda and type(x) in _PLAIN and not torch.compiler.is_compiling() and not torch.is_autocast_enabled():
+        return _lib._ext or _lib.extension()
+    return None
+
+
+_PLAIN = (torch.Tensor, nn.Parameter)
+_EPS = torch.finfo(torch.float32).eps   # F.rms_norm's default for bf16 and fp32
+
+
+def _norm_kernel_takes(x: torch.Tensor) -> bool:
+    return 0 < x.size(-1) <= 4096 and x.size(-1) % 4 == 0 and x.numel() > 0
+
+
 def RT_norm(x: torch.Tensor) -> torch.Tensor:
+    ext = _fused(x)
+    if ext is not None and _norm_kernel_takes(x):
+        return ext.rms_norm(x, _EPS)
     return F.rms_norm(x, (x.size(-1),))
+
+
+def _add_norm(x: torch.Tensor, delta: torch.Tensor):
+    """``x + delta`` and its normalisation."""
+    ext = _fused(x)
+    if ext is not None and delta.dtype is torch.bfloat16 and delta.shape == x.shape and _norm_kernel_takes(x):
+        return ext.add_rms_norm(x, delta, _EPS)
+    x = x + delta
+    return x, RT_norm(x)
 
 
 class Rotary(nn.Module):
@@ -74,7 +104,11 @@ class RT_CausalSelfAttention(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         B, T, D = x.shape
-        q, k, v = self.c_qkv(x).view(B, T, 3, self.n_head, D // self.n_head).unbind(2)
+        qkv = self.c_qkv(x)
+        ext = _fused(qkv)
+        if ext is not None and D == 64 * self.n_head and 0 < T * 3 * D < 1 << 29 and B > 0:
+            return self.c_proj(ext.causal_attention(qkv, self.rotary.inv_freq, self.n_head, _EPS))
+        q, k, v = qkv.view(B, T, 3, self.n_head, D // self.n_head).unbind(2)
         q, k = RT_norm(q), RT_norm(k)
         q, k = self.rotary(q), self.rotary(k)
         y = F.scaled_dot_product_attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), is_causal=True)
@@ -88,7 +122,9 @@ class RT_MLP(nn.Module):
         self.c_proj = RT_CastedLinear(4 * dim, dim, config)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.c_proj(F.relu(self.c_fc(x)).square())
+        h = self.c_fc(x)
+        ext = _fused(h)
+        return self.c_proj(F.relu(h).square() if ext is None else ext.relu_square(h))
 
 
 class RT_Block(nn.Module):
@@ -98,8 +134,8 @@ class RT_Block(nn.Module):
         self.mlp = RT_MLP(config.n_embd, config)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        x = x + self.attn(RT_norm(x))
-        return x + self.mlp(RT_norm(x))
+        x, h = _add_norm(x, self.attn(RT_norm(x)))
+        return x + self.mlp(h)
 
 
 class RT_GPT(nn.Module):
@@ -122,5 +158,9 @@ class RT_GPT(nn.Module):
         x = RT_norm(x.to(self.h[0].mlp.c_fc.weight_coef.dtype))
         for block in self.h:
             x = block(x)
-        logits = self.lm_head(RT_norm(x)).float()
+        logits = self.lm_head(RT_norm(x))
+        ext = _fused(logits)
+        if ext is not None and logits.size(-1) % 8 == 0 and logits.numel() and target.dtype is torch.int64:
+            return ext.cross_entropy(logits.view(-1, logits.size(-1)), target.view(-1), -100)
+        logits = logits.float()
         return F.cross_entropy(logits.view(-1, logits.size(-1)), target.view(-1))

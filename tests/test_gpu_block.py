@@ -1,0 +1,149 @@
+"""The kernels around a block's linears (randumb_amd/csrc/rdb_block.hip, rdb_attention.hip) against the stock operators they
+replace, in fp32 or fp64 on the same bf16 inputs, at sizes around their tiles' edges."""
+import math
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+EPS = torch.finfo(torch.float32).eps
+
+
+@pytest.fixture(scope="module")
+def ext():
+    from randumb_amd import _lib
+
+    return _lib.extension()
+
+
+def rel(a, b):
+    a, b = a.detach().double(), b.detach().double()
+    return float((a - b).norm() / b.norm().clamp_min(1e-30))
+
+
+def bf16(g, *shape, scale=1.0):
+    return (torch.randn(*shape, generator=g, device="cuda") * scale).bfloat16()
+
+
+@pytest.mark.parametrize("rows,dim", [(1, 4), (3, 64), (5, 260), (130, 768), (7, 1024), (2, 2052), (3, 4096)])
+def test_rms_norm_and_residual(ext, rows, dim):
+    print(f"case rms norm {rows} x {dim}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(dim)
+    x, d, dy, ds = (bf16(g, rows, dim, scale=s) for s in (1.0, 0.5, 1.0, 1.0))
+    leaves = [t.clone().requires_grad_() for t in (x, d)]
+    ref = [t.double().requires_grad_() for t in (x, d)]
+    s, y = ext.add_rms_norm(*leaves, EPS)
+    assert torch.equal(s, x + d)
+    rs = (ref[0] + ref[1])
+    rs = rs + (s.double() - rs).detach()   # the sum is rounded to bf16 before it is normalised
+    ry = F.rms_norm(rs, (dim,), eps=EPS)
+    assert rel(y, ry) < 3e-3
+    got = torch.autograd.grad([s, y], leaves, [ds, dy])
+    want = torch.autograd.grad([rs, ry], ref, [ds.double(), dy.double()])
+    assert torch.equal(got[0], got[1]) and rel(got[0], want[0]) < 5e-3
+    p, q = x.clone().requires_grad_(), x.double().requires_grad_()
+    y, ry = ext.rms_norm(p, EPS), F.rms_norm(q, (dim,), eps=EPS)
+    assert rel(y, ry) < 3e-3
+    if dim > 4:   # with so few values the gradient is what is left of a cancellation
+        assert rel(torch.autograd.grad(y, p, dy)[0], torch.autograd.grad(ry, q, dy.double())[0]) < 5e-3
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 2047, 5000, 1 << 20])
+def test_relu_square_is_the_stock_chain_bit_for_bit(ext, n):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, dy = bf16(g, n), bf16(g, n)
+    x[0] = math.nan
+    a, b = x.clone().requires_grad_(), x.clone().requires_grad_()
+    ya, yb = ext.relu_square(a), F.relu(b).square()
+    assert torch.equal(ya.nan_to_num(7), yb.nan_to_num(7)) and bool(ya[0].isnan())
+    ga, gb = torch.autograd.grad(ya, a, dy)[0], torch.autograd.grad(yb, b, dy)[0]
+    assert torch.equal(ga.nan_to_num(7), gb.nan_to_num(7))
+
+
+@pytest.mark.parametrize("rows,classes", [(1, 8), (3, 64), (130, 2056), (1025, 4096), (64, 50304)])
+def test_cross_entropy(ext, rows, classes):
+    print(f"case cross entropy {rows} x {classes}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(classes)
+    x = bf16(g, rows, classes, scale=3.0)
+    t = torch.randint(0, classes, (rows,), generator=g, device="cuda")
+    if rows > 2:
+        t[1] = -100
+        x[2, : classes // 2] = -math.inf
+        t[2] = classes - 1
+    a, b = x.clone().requires_grad_(), x.double().requires_grad_()
+    la, lb = ext.cross_entropy(a, t, -100), F.cross_entropy(b, t)
+    assert la.dtype == torch.float32 and la.shape == () and abs(float(la.detach()) - float(lb.detach())) < 1e-5 * abs(float(lb.detach()))
+    ga, gb = torch.autograd.grad(la * 3, a)[0], torch.autograd.grad(lb * 3, b)[0]
+    assert rel(ga, gb) < 3e-3
+    if rows > 2:
+        assert not bool(ga[1].any())
+    assert torch.equal(torch.autograd.grad(ext.cross_entropy(a, t, -100) * 3, a)[0], ga)
+    assert bool(ext.cross_entropy(x, torch.full_like(t, -100), -100).isnan())   # no row counts, as in the stock operator
+    assert bool(ext.cross_entropy(x, torch.full_like(t, classes), -100).isnan())
+
+
+def _attention(qkv, inv_freq, H):
+    """The stock operators of RT_CausalSelfAttention, in qkv's precision, with q, k rounded to bf16 as they are there."""
+    from randumb_amd.gpt import Rotary
+
+    B, T, D3 = qkv.shape
+    q, k, v = qkv.view(B, T, 3, H, 64).unbind(2)
+
+    def r16(t):   # value rounded to bf16, gradient passed on
+        return t + (t.detach().bfloat16().to(t.dtype) - t.detach())
+
+    freqs = torch.outer(torch.arange(T, device=qkv.device), inv_freq)
+    cos, sin = freqs.cos().to(qkv.dtype)[None, :, None, :], freqs.sin().to(qkv.dtype)[None, :, None, :]
+
+    def rot(x):
+        x = r16(F.rms_norm(x, (64,), eps=EPS))
+        x1, x2 = x.chunk(2, dim=3)
+        return r16(torch.cat((x1 * cos + x2 * sin, x2 * cos - x1 * sin), 3))
+
+    q, k = rot(q).transpose(1, 2), rot(k).transpose(1, 2)
+    s = (q @ k.transpose(-1, -2).contiguous()) / 8.0
+    s = s.masked_fill(torch.ones(T, T, dtype=torch.bool, device=qkv.device).triu(1), -math.inf)
+    assert Rotary is not None
+    return (s.softmax(-1) @ v.transpose(1, 2).contiguous()).transpose(1, 2).reshape(B, T, H * 64)
+
+
+@pytest.mark.parametrize("B,T,H,inv", [(1, 1, 1, "bf16"), (2, 31, 3, "fp32"), (1, 64, 2, "bf16"), (1, 65, 8, "bf16"), (2, 127, 1, "bf16"), (1, 129, 5, "fp32"),
+                                       (2, 200, 4, "bf16"), (1, 384, 2, "bf16"), (1, 1000, 3, "bf16")])
+def test_causal_attention(ext, B, T, H, inv):
+    print(f"case attention B={B} T={T} H={H} {inv}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    qkv = bf16(g, B, T, 3 * H * 64, scale=0.7)
+    dy = bf16(g, B, T, H * 64)
+    f = (1.0 / 10000.0) ** (torch.arange(0, 64, 2, device="cuda") / 64)
+    f = f.bfloat16() if inv == "bf16" else f
+    a, b = qkv.clone().requires_grad_(), qkv.double().requires_grad_()
+    ya, yb = ext.causal_attention(a, f, H, EPS), _attention(b, f, H)
+    assert ya.shape == (B, T, H * 64) and rel(ya, yb) < 5e-3
+    ga, gb = torch.autograd.grad(ya, a, dy)[0], torch.autograd.grad(yb, b, dy.double())[0]
+    for part, (x, w) in enumerate(zip(ga.view(B, T, 3, -1).unbind(2), gb.view(B, T, 3, -1).unbind(2))):
+        if T > 1 or part == 2:   # with one token there is no gradient in q and k but rounding
+            assert rel(x, w) < 1.5e-2, part
+    y2 = ext.causal_attention(a, f, H, EPS)
+    assert torch.equal(y2, ya) and torch.equal(torch.autograd.grad(y2, a, dy)[0], ga)
+
+
+def test_model_with_and_without_the_fused_kernels(ext, monkeypatch):
+    from randumb_amd import gpt
+
+    torch.manual_seed(0)
+    with torch.device("cuda"):
+        model = gpt.RT_GPT(gpt.RT_GPTConfig(int_dim_gen=iter([32] * 8), seed_gen=iter(range(8)), vocab_size=512, n_layer=2, n_head=2, n_embd=128)).bfloat16()
+    ids = torch.randint(0, 512, (2, 97), device="cuda")
+    out = []
+    for fused in (True, False):
+        if not fused:
+            monkeypatch.setattr(gpt, "_fused", lambda x: None)
+        model.zero_grad(set_to_none=True)
+        loss = model(ids[:, :-1].contiguous(), ids[:, 1:].contiguous())
+        loss.backward()
+        out.append([loss.detach()] + [p.grad for p in model.parameters() if p.grad is not None])
+    assert len(out[0]) == len(out[1]) == 1 + 8 + 2
+    assert abs(float(out[0][0]) - float(out[1][0])) < 1e-3 * float(out[1][0])
+    for x, y in zip(out[0], out[1]):
+        assert rel(x, y) < 2e-2

@@ -16,6 +16,8 @@
 
 namespace rdb {
 
+int num_compute_units();   // rdb_error.hip
+
 constexpr float INV_2_31 = 4.656612873077392578125e-10f;
 constexpr int F_BK = 64;
 
@@ -39,6 +41,14 @@ struct ZParams {
     unsigned long long *sync;   // NULL, or slots [tiles_t][tiles_m + 1]: a block sets its slot to sync_tag when its tile is in memory;
                                 // slot tiles_m of a token tile counts its consumers and is cleared by the block of coefficient tile 0
     unsigned long long sync_tag;
+    // The contraction is added up in `ranges` ranges of range_stages stages of 64 features, range by range, whoever computes them.
+    // part == NULL: every block runs its tile's ranges one after the other.  Otherwise the grid holds a block per tile and range,
+    // range by range; the blocks of the last range of a tile wait for the others' sums.  A token tile's sums lie in its own
+    // rows of y, which nobody writes before they have been read (a multiplying block waits for all of its tokens' z):
+    // [coefficient tile][range][token of the tile][32] floats, and behind them, at the end of the rows, a tag for each.
+    int ranges, range_stages;
+    char *part;
+    SyncWait sync_wait;
 };
 
 // Eight waves, two to a SIMD: the tile's noise is hashed once per stage by all 512 threads (4 values each) on the vector ALU,
@@ -47,8 +57,10 @@ struct ZParams {
 // barrier.  Written without the 256-thread tile engine; the LDS layouts and fragment reads are the engine's (OperandTile).
 constexpr int KZ_THREADS = 512;
 
-// `block` of `nblocks`: index of this block among the blocks that run this body; all KZ_THREADS threads must call.
-__device__ __forceinline__ void z_block(const ZParams &p, unsigned char *smem_raw, int block, int nblocks)
+// `block` of `nblocks`: index of this block among the blocks that run this body; all KZ_THREADS threads must call.  RANGES: the
+// contraction may be in several ranges; a kernel of its own for the ordinary case, whose 128 registers let two blocks share a
+// compute unit (tiles by the hundred: 4096 tokens x 4096 features, k = 1024: 75 us, 105 with the registers of the other).
+template <bool RANGES> __device__ __forceinline__ void z_block(const ZParams &p, unsigned char *smem_raw, int block, int nblocks)
 {
     bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
@@ -84,7 +96,9 @@ __device__ __forceinline__ void z_block(const ZParams &p, unsigned char *smem_ra
         }
     };
     // work item = (token tile, coefficient tile), coefficient tile fastest: neighbours share the x tile
-    const int w = xcd_work_item(block, p.tiles_m * p.tiles_t);
+    const bool part = RANGES && p.part;
+    const int range_blocks = part ? nblocks / p.ranges : nblocks, my_range = RANGES ? block / range_blocks : 0;
+    const int w = xcd_work_item(block - my_range * range_blocks, p.tiles_m * p.tiles_t);
     if (w >= p.tiles_m * p.tiles_t) {
         finish_units();
         return;
@@ -93,7 +107,7 @@ __device__ __forceinline__ void z_block(const ZParams &p, unsigned char *smem_ra
     // A replay of a recorded launch carries the tag it was recorded with.  The consumers clear the slots when all of them are
     // past their wait; should one of them have given up in an earlier replay, a slot may still hold the tag: take it back
     // before this tile is touched.
-    if (p.sync && t == 0)
+    if (p.sync && t == 0 && (!part || my_range == p.ranges - 1))
         __hip_atomic_store(p.sync + (int64_t)(w / p.tiles_m) * (p.tiles_m + 1) + w % p.tiles_m, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     RDB_STAMP(0);
     typedef OperandTile<KZ_BM, F_BK, K_CONT> TN;   // noise tile: rows = coefficients, contraction = input features
@@ -133,16 +147,8 @@ __device__ __forceinline__ void z_block(const ZParams &p, unsigned char *smem_ra
         v.y = f32x2_to_bf16x2((float)(int32_t)sq5_tail(f0 + 2u * PN1), (float)(int32_t)sq5_tail(f0 + 3u * PN1));
         *reinterpret_cast<uint2 *>(buf + nlds) = v;
     };
-    f32x16 acc = zero16();
+    f32x16 acc = zero16(), sum = zero16();
     f32x4 rx[2][XP];
-    {
-        f32x4 rx0[XP];
-        load_x(rx0, 0);
-        load_x(rx[1], 1);
-        load_x(rx[0], 2);
-        hash_noise(lds, 0);
-        store_x(lds, rx0);
-    }
     RDB_STAMP(1);
     auto stage_body = [&](int s, int u, bool more) {   // stage s in LDS buffer u (= s % 2); slot (u ^ 1) of rx holds stage s + 1
         bf16_t *cur = lds + u * STAGE, *oth = lds + (u ^ 1) * STAGE;
@@ -161,15 +167,78 @@ __device__ __forceinline__ void z_block(const ZParams &p, unsigned char *smem_ra
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks], fb[ks], acc, 0, 0, 0);
     };
-    int s = 0;
-    for (; s + 2 < nstage; s += 2) {
-        stage_body(s, 0, true);
-        stage_body(s + 1, 1, true);
+    for (int rg = my_range; rg < (!RANGES || part ? my_range + 1 : p.ranges); ++rg) {
+        int s = RANGES ? rg * p.range_stages : 0;
+        const int s_end = RANGES ? min(nstage, s + p.range_stages) : nstage;
+        {
+            f32x4 rx0[XP];
+            load_x(rx0, s);
+            load_x(rx[1], s + 1);
+            load_x(rx[0], s + 2);
+            hash_noise(lds, s);
+            store_x(lds, rx0);
+        }
+        for (; s + 2 < s_end; s += 2) {
+            stage_body(s, 0, true);
+            stage_body(s + 1, 1, true);
+        }
+        stage_body(s, 0, s + 1 < s_end);
+        if (s + 1 < s_end) stage_body(s + 1, 1, false);
+        if (RANGES && !part) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) sum[j] += acc[j];
+            acc = zero16();
+            __syncthreads();   // the next range begins by writing the buffer just read
+        }
     }
-    stage_body(s, 0, s + 1 < nstage);
-    if (s + 1 < nstage) stage_body(s + 1, 1, false);
+    if (RANGES && !part) acc = sum;
     finish_units();
     __syncthreads();   // the last stage's fragment reads are done: the tile buffers may be reused
+    if (part) {
+        const int rows = min(KZ_BT, p.tokens - tok0), others = p.ranges - 1, mt = w % p.tiles_m;
+        char *base = p.part + (int64_t)tok0 * p.out_f * 2;
+        unsigned long long *tags = reinterpret_cast<unsigned long long *>(base + (int64_t)rows * p.out_f * 2) - (int64_t)p.tiles_m * others + mt * others;
+        const __amdgpu_buffer_rsrc_t rs_p = __builtin_amdgcn_make_buffer_rsrc(base, 0, p.tiles_m * others * rows * 128, 0x00020000);
+        const int row = wave * 32 + (lane & 31);
+        auto at = [&](int rg, int jq) { return row < rows ? (uint32_t)(((mt * others + rg) * rows + row) * 128 + (8 * jq + 4 * (lane >> 5)) * 4) : BUFFER_OOB; };
+        if (my_range < others) {
+#pragma unroll
+            for (int jq = 0; jq < 4; ++jq) {
+                const f32x4 v = {acc[jq * 4], acc[jq * 4 + 1], acc[jq * 4 + 2], acc[jq * 4 + 3]};
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v), rs_p, (int)at(my_range, jq), 0, SCOPE_DEVICE);
+            }
+            publish_tag(tags + my_range, p.sync_tag);
+            return;
+        }
+        volatile int *verdict = reinterpret_cast<volatile int *>(smem_raw);
+        if (wave == 0) {
+            const bool there = await_tags(tags, others, p.sync_tag, p.sync_wait);
+            if (lane == 0) *verdict = there ? 1 : 0;
+        }
+        __syncthreads();
+        if (*verdict) {
+            for (int r0 = 0; r0 < others; r0 += 4) {   // four ranges' loads in flight; added in range order, this block's own last
+                f32x4 v[4][4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int jq = 0; jq < 4; ++jq)
+                        v[i][jq] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_p, (int)(r0 + i < others ? at(r0 + i, jq) : BUFFER_OOB), 0,
+                                                                                                   SCOPE_DEVICE));
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < 16; ++j)
+                        if (r0 + i < others) sum[j] += v[i][j >> 2][j & 3];
+            }
+#pragma unroll
+            for (int j = 0; j < 16; ++j) acc[j] = sum[j] + acc[j];
+        } else {   // gave up: the tile of z becomes NaN, and with it everything computed from it
+#pragma unroll
+            for (int j = 0; j < 16; ++j) acc[j] = __uint_as_float(0x7fc00000u);
+        }
+        __syncthreads();   // the verdict has been read: its word may be overwritten
+    }
     RDB_STAMP(2);
     // The tile D[a = coefficient][b = token] goes to LDS once, as bf16 rows of tokens (LD elements apart), and leaves in
     // up to two orders.  Rows of tokens past the end and coefficients past k hold zeros or finite values: every byte of the
@@ -222,10 +291,10 @@ __device__ __forceinline__ void z_block(const ZParams &p, unsigned char *smem_ra
     RDB_STAMP(3);
 }
 
-__global__ __launch_bounds__(KZ_THREADS, 1) void factored_z_kernel(ZParams p)
+template <bool RANGES> __global__ __launch_bounds__(KZ_THREADS, 1) void factored_z_kernel(ZParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    z_block(p, smem_raw, blockIdx.x, gridDim.x);
+    z_block<RANGES>(p, smem_raw, blockIdx.x, gridDim.x);
 }
 
 // ----------------------------------------------------------------------------------------------- y = z . C^T
@@ -287,7 +356,7 @@ template <int KG, bool BIAS> __global__ __launch_bounds__(ST_THREADS, 1) void fa
     static_assert(KZ_THREADS == ST_THREADS && KZ_BT == ST_BT, "one block size and one token tile for both kinds of block");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     if ((int)blockIdx.x < p.z_blocks)
-        z_block(p.z, smem_raw, blockIdx.x, p.z_blocks);
+        z_block<true>(p.z, smem_raw, blockIdx.x, p.z_blocks);
     else
         stationary_block<KG, BIAS, false, true>(p.y, smem_raw, blockIdx.x - p.z_blocks);
 }
@@ -329,6 +398,23 @@ void dc_params_from_state(DcParams &p, const void *state, const rdb_linear_desc 
 int linear_fwd_projected(void *y, int64_t ldy, const void *state, const void *coef, const void *bias, const rdb_linear_desc *d, int num_cus,
                          hipStream_t s);
 
+// Ranges of the projection's contraction.  A tile's block walks over all of in_f, half a microsecond per 64 features: with fewer
+// tiles than compute units the others stand idle meanwhile (2000 tokens x 4096 features, k = 256: 64 tiles of 64 stages).  So as
+// many ranges as leave a unit for every block, of at least KZ_MIN_STAGES stages: below that the wait for the others' sums and
+// fetching them (some 4 us) costs what the shorter loop saves.  The sums need (ranges - 1) * kpad * 4 bytes of a token's out_f * 2.
+// The numbers depend on the layer alone, so that the same sums in the same order come out wherever they are computed.
+constexpr int KZ_MIN_STAGES = 8, KZ_MAX_RANGES = 16;
+static void z_ranges(const rdb_linear_desc *d, int tiles, int &ranges, int &range_stages)
+{
+    const int nstage = (int)cdiv(d->in_f, F_BK), kpad = (int)cdiv(d->k, 64) * 64;
+    int64_t r = std::min<int64_t>(std::min<int64_t>(num_compute_units() / tiles, nstage / KZ_MIN_STAGES), KZ_MAX_RANGES);
+    r = std::min<int64_t>(r, 1 + (d->out_f * 2 - 64) / (kpad * 4 + kpad / 4));
+    if (r < 1) r = 1;
+    range_stages = (int)cdiv(nstage, r);
+    range_stages += range_stages & 1;   // the stages alternate between two buffers, beginning with the first
+    ranges = (int)cdiv(nstage, range_stages);
+}
+
 static bool fill_z_params(ZParams &p, void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d)
 {
     const ProjLayout L = proj_layout(d);
@@ -354,19 +440,47 @@ static bool fill_z_params(ZParams &p, void *state, const void *x, int64_t ldx, c
     p.tiles_t = (int)cdiv(d->tokens, KZ_BT);
     p.sync = nullptr;
     p.sync_tag = 0;
+    p.part = nullptr;
+    z_ranges(d, p.tiles_m * p.tiles_t, p.ranges, p.range_stages);
+    return true;
+}
+
+// Spreads the ranges of a split contraction over blocks of their own, with the sums on the way in y's rows (contiguous, not yet
+// written).  False when there is nothing to spread, or y is not the place.
+static bool spread_ranges(ZParams &p, void *state, void *y, int64_t ldy, const rdb_linear_desc *d, int *rc)
+{
+    *rc = RDB_OK;
+    if (p.ranges <= 1 || !y || ldy != d->out_f || !aligned16(y) || !one_launch_mode()) return false;
+    p.part = static_cast<char *>(y);
+    if (!p.sync_tag) p.sync_tag = next_sync_tag();
+    p.sync_wait.err = reinterpret_cast<unsigned int *>(state) + 1;
+    p.sync_wait.polls = SYNC_SPIN_LIMIT;
+    *rc = sync_giveups_ptr(&p.sync_wait.giveups);
     return true;
 }
 
 static size_t z_smem() { return engine_smem<KZ_BM, KZ_BT, F_BK, K_CONT, K_CONT>(); }
 
-int linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, hipStream_t s)
+// y: NULL, or the rows of the forward product to come, free to hold sums on the way
+static int launch_z(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, hipStream_t s)
 {
     ZParams p;
+    int rc;
     if (!fill_z_params(p, state, x, ldx, coef, d)) return RDB_E_UNSUPPORTED;
+    const bool spread = spread_ranges(p, state, y, ldy, d, &rc);
+    if (rc) return rc;
     const size_t smem = z_smem();
-    if (int rl = reserve_lds(reinterpret_cast<const void *>(factored_z_kernel), smem, "factored_z_kernel")) return rl;
-    factored_z_kernel<<<xcd_grid_size(p.tiles_m * p.tiles_t), KZ_THREADS, smem, s>>>(p);
+    const void *fn = p.ranges > 1 ? (const void *)factored_z_kernel<true> : (const void *)factored_z_kernel<false>;
+    if (int rl = reserve_lds(fn, smem, "factored_z_kernel")) return rl;
+    const unsigned grid = xcd_grid_size(p.tiles_m * p.tiles_t) * (spread ? p.ranges : 1);
+    if (p.ranges > 1) factored_z_kernel<true><<<grid, KZ_THREADS, smem, s>>>(p);
+    else factored_z_kernel<false><<<grid, KZ_THREADS, smem, s>>>(p);
     return check_launch("factored_z_kernel");
+}
+
+int linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, hipStream_t s)
+{
+    return launch_z(state, x, ldx, coef, nullptr, 0, d, s);
 }
 
 // The forward product's parameters when the contraction of a token fits in registers (z in fragment order); returns the
@@ -407,7 +521,7 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
         // check the second call's conditions before the first launch, so that a refusal leaves nothing half done
         if (d->coef_dtype != RDB_BF16 || ldy % 8 || !aligned16(y) || !aligned16(coef)) return RDB_E_UNSUPPORTED;
         if (((uintptr_t)bias & 7) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
-        if (int rc = linear_project(state, x, ldx, with_ct ? coef : nullptr, d, s)) return rc;
+        if (int rc = launch_z(state, x, ldx, with_ct ? coef : nullptr, y, ldy, d, s)) return rc;
         return linear_fwd_projected(y, ldy, state, coef, bias, d, num_cus, s);
     }
     const ProjLayout L = proj_layout(d);
@@ -419,7 +533,10 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
     p.y.sync_wait.err = reinterpret_cast<unsigned int *>(state) + 1;
     p.y.sync_wait.polls = SYNC_SPIN_LIMIT;
     if (int rc = sync_giveups_ptr(&p.y.sync_wait.giveups)) return rc;
-    p.z_blocks = xcd_grid_size(p.z.tiles_m * p.z.tiles_t);
+    int rc;
+    const bool spread = spread_ranges(p.z, state, y, ldy, d, &rc);
+    if (rc) return rc;
+    p.z_blocks = xcd_grid_size(p.z.tiles_m * p.z.tiles_t) * (spread ? p.z.ranges : 1);
     const int kg = (int)cdiv(d->k, 64);
     if (bias) {
         switch (kg) {

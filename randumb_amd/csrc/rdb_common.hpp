@@ -42,6 +42,34 @@ __device__ __forceinline__ uint32_t sq5_tail(uint32_t b)
     return b;
 }
 
+// The same for kernels that do nothing but hash, with six waves a SIMD or more.  An exclusive or that the compiler cannot merge with the
+// addition that follows: v_xad_u32 occupies the vector ALU longer than v_xor_b32 and v_add_u32 together when other waves' instructions
+// are there to issue beside those (4.4 against 2 x 2.6 clocks a wave; a hash and its use: 2.79 -> 3.03 T/s).  In the kernels that
+// hash between matrix instructions, with two waves a SIMD, the merged form is the faster one (8192 x 768 -> 3072 random-bias shares: 3 %).
+__device__ __forceinline__ uint32_t sq5_xor(uint32_t a, uint32_t b)
+{
+    uint32_t r;
+    asm("v_xor_b32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+// ... up to the last round's shift
+__device__ __forceinline__ uint32_t sq5_tail_apart_but_last(uint32_t b)
+{
+    b = sq5_xor(b, b >> 9);
+    b += SQ5_N2;
+    b ^= (b >> 11);
+    b *= SQ5_N3;
+    b = sq5_xor(b, b >> 13);
+    b += SQ5_N4;
+    b ^= (b >> 15);
+    return b * SQ5_N5;
+}
+__device__ __forceinline__ uint32_t sq5_tail_apart(uint32_t b)
+{
+    b = sq5_tail_apart_but_last(b);
+    return b ^ (b >> 17);
+}
+
 __device__ __forceinline__ uint32_t sq5_bits(uint32_t idx, uint32_t seed) { return sq5_tail(idx * SQ5_N1 + seed); }
 
 // int32 reinterpretation -> fp32 (round to nearest even) -> exact scale by 2^-31

@@ -40,45 +40,52 @@ __global__ __launch_bounds__(NT) void sq5_fill_1d_kernel(float *__restrict__ out
 }
 
 // =============================================================================================== forward
-// Vector-coef materialise / embedding gather: one thread per output element, coef broadcast from LDS,
-// serial fp32 FMA over m (the order the reference's CUDA kernel uses, rten.cu:101-104).
+// Vector-coef materialise / embedding gather: one thread per output element, coef broadcast from LDS, serial fp32 FMA over m (the
+// order the reference's CUDA kernel uses, rten.cu:101-104).  Bound by the hash on the vector ALU.
 // GATHER = false: a = (n % Q)*sQ + (n / Q)*sP                       (RandumbTensor.py:264)
 // GATHER = true : a = idx[n / Q]*Q + n % Q   (Q = rowsize)          (RandumbTensor.py:1029)
+// A thread's terms are one chain of dependent instructions, on purpose: eight waves a SIMD fill each other's gaps, and two waves'
+// instructions can issue together where one wave's cannot (several elements a thread, or their terms interleaved: 2.6 - 2.8
+// Thash/s; this form: 3.0 at 768 x 3072 elements, k = 256, 222 -> 200 us, 3.1 at k = 1024).  Also measured: the terms as bytes of an 8-bit
+// matrix operand, without conversion and multiplication on the vector ALU (v_mfma_i32_16x16x64_i8): 229 us.
 constexpr int COEF_CHUNK = 2048;
 
-template <bool GATHER>
-__global__ __launch_bounds__(NT) void materialize_vec_kernel(float *__restrict__ out, const void *__restrict__ coef,
-                                                             int coef_dtype, int64_t k, int64_t Nw, int64_t Q,
-                                                             int64_t sP, int64_t sQ, uint32_t seed,
-                                                             const void *__restrict__ scale_bias,
-                                                             const int64_t *__restrict__ idx)
+struct MatVecParams {
+    float *out;
+    const void *coef, *scale_bias;
+    const int64_t *idx;
+    int64_t k, Nw, Q, sP, sQ;
+    int coef_dtype, narrow, contiguous;   // narrow: element numbers fit 32 bits; contiguous: element n has offset n
+    uint32_t seed;
+};
+
+template <bool GATHER> __global__ __launch_bounds__(NT) void materialize_vec_kernel(MatVecParams p)
 {
     __shared__ float cs[COEF_CHUNK];
     const int64_t n = (int64_t)blockIdx.x * NT + threadIdx.x;
-    const bool live = n < Nw;
-    uint32_t a = 0;
-    if (live) {
-        const int64_t p = n / Q, q = n - p * Q;
-        a = GATHER ? (uint32_t)(idx[p] * Q + q) : (uint32_t)(q * sQ + p * sP);
+    const bool live = n < p.Nw;
+    uint32_t a = (uint32_t)n;
+    if (live && (GATHER || !p.contiguous)) {
+        const int64_t r = p.narrow ? (int64_t)((uint32_t)n / (uint32_t)p.Q) : n / p.Q, q = n - r * p.Q;
+        a = GATHER ? (uint32_t)(p.idx[r] * p.Q + q) : (uint32_t)(q * p.sQ + r * p.sP);
     }
-    uint32_t first = a * PN1 + seed;  // first-round value for m = 0; +N1 per step of m
+    uint32_t first = a * PN1 + p.seed;  // first-round value for m = 0; +N1 per step of m
     float acc = 0.0f;
-    for (int64_t m0 = 0; m0 < k; m0 += COEF_CHUNK) {
-        const int cnt = (int)((k - m0) < COEF_CHUNK ? (k - m0) : COEF_CHUNK);
+    for (int64_t m0 = 0; m0 < p.k; m0 += COEF_CHUNK) {
+        const int cnt = (int)((p.k - m0) < COEF_CHUNK ? (p.k - m0) : COEF_CHUNK);
         __syncthreads();
-        for (int j = threadIdx.x; j < cnt; j += NT) cs[j] = load_as_f32(coef, coef_dtype, m0 + j);
+        for (int j = threadIdx.x; j < cnt; j += NT) cs[j] = load_as_f32(p.coef, p.coef_dtype, m0 + j);
         __syncthreads();
         if (live) {
-#pragma unroll 4
             for (int j = 0; j < cnt; ++j) {
-                acc = fmaf(sq5_unit(sq5_tail(first)), cs[j], acc);
+                acc = fmaf(sq5_unit(sq5_tail_apart(first)), cs[j], acc);
                 first += SQ5_N1;
             }
         }
     }
     if (live) {
-        if (scale_bias) acc += load_as_f32(scale_bias, coef_dtype, 0) * noise1d(a, seed);
-        out[n] = acc;
+        if (p.scale_bias) acc += load_as_f32(p.scale_bias, p.coef_dtype, 0) * noise1d(a, p.seed);
+        p.out[n] = acc;
     }
 }
 
@@ -154,67 +161,201 @@ __global__ __launch_bounds__(NT) void materialize_mat_tiled_kernel(float *__rest
 }
 
 // =============================================================================================== backward
+// ----------------------------------------------------------------------------------------------- sums over elements on the matrix cores
+// The gradient's terms noise(a, m) d[a] are summed over the elements a: with a lane per coefficient every term would fetch its d
+// and its first-round value from LDS (2.1 - 2.4 Thash/s, as a plain chain or interleaved).  Taken off the vector ALU instead: a
+// hashed 32-bit integer is, as it lies in its register, four bytes of an 8-bit matrix operand.  d becomes an integer q of 39 bits
+// relative to the largest of the block's span (below 2^-39 of it is dropped; fp32 sums drop more at every addition), in five
+// signed base-256 digits, and
+//     sum n q = sum over s of 256^s . sum over (element, byte j of n) of byte_j(n) . digit_(s-j)(q)
+// is one v_mfma_i32_16x16x64_i8 per 16 elements x 16 coefficients: rows = s (0 .. 7, twice), columns = coefficients, contraction =
+// (element, byte).  The 32-bit sums are exact for up to 2^14 elements; they are put together in fp64 and rounded once.  (Bytes 0 .. 2 of n
+// are unsigned where the instruction takes signed ones: n ^ 0x00808080 gives n - 128 (1 + 2^8 + 2^16), and 8421504 . sum q is
+// added back.)  13 vector instructions a term and no LDS read: 768 x 3072 elements, k = 256: 250 -> 204 us (2.95 Thash/s), and
+// 33 -> 4 for the partial rows' sum.
+typedef int q8x4 __attribute__((ext_vector_type(4)));
+constexpr double Q_OFFSET = 8421504.0;   // 128 (1 + 2^8 + 2^16)
+
+// b: first-round value
+__device__ __forceinline__ int q8_hash(uint32_t b)
+{
+    b = sq5_tail_apart_but_last(b);
+    return (int)__builtin_amdgcn_bitop3_b32(b, b >> 17, 0x00808080u, 0x96);   // three-way exclusive or in one instruction
+}
+
+// p with which values of at most the magnitude behind `top` (the largest |v| as bits, finite), times 2^p, stay below 2^38
+__device__ __forceinline__ int q8_exponent(uint32_t top)
+{
+    if (top == 0) return 0;
+    const int e = (int)(top >> 23);
+    return e ? 38 - (e - 126) : 38 - (-117 - __clz((int)top));   // |v| < 2^(e - 126); denormals: 2^(32 - clz - 149)
+}
+__device__ __forceinline__ double pow2(int p) { return __longlong_as_double((long long)(p + 1023) << 52); }
+
+// q = v 2^p and the eight windows of its digits: byte j of win[s] is digit s - j
+__device__ __forceinline__ long long q8_windows(float v, double scale, uint32_t (&win)[8])
+{
+    const long long q = __double2ll_rn((double)v * scale);
+    const unsigned long long w = ((unsigned long long)q + 0x8080808080ull) ^ 0x8080808080ull;
+    const uint32_t lo = __builtin_bswap32((uint32_t)w), hi = (uint32_t)(w >> 32) << 24;
+    win[7] = hi;
+    win[6] = __builtin_amdgcn_alignbyte(lo, hi, 1);
+    win[5] = __builtin_amdgcn_alignbyte(lo, hi, 2);
+    win[4] = __builtin_amdgcn_alignbyte(lo, hi, 3);
+    win[3] = lo;
+    win[2] = lo >> 8;
+    win[1] = lo >> 16;
+    win[0] = lo >> 24;
+    return q;
+}
+
+// A result's rows are 4 (lane / 16) + j (r and r + 8 the same): put together.  Lanes 0 .. 31 take the columns of one accumulator, lanes
+// 32 .. 63 those of the other; the two halves of a column meet across 16 lanes.
+__device__ __forceinline__ double q8_total(const q8x4 &low, const q8x4 &high)
+{
+    const bool second = threadIdx.x & 32;
+    double v = 0.0;
+#pragma unroll
+    for (int j = 3; j >= 0; --j) v = v * 256.0 + (double)(second ? high[j] : low[j]);
+    if (threadIdx.x & 16) v *= 4294967296.0;
+    const long long bits = __double_as_longlong(v);
+    const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)bits, (uint32_t)bits, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(bits >> 32), (uint32_t)(bits >> 32), false, false);
+    return __longlong_as_double(((long long)hi[0] << 32) | lo[0]) + __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+}
+
+// Largest |v| (as bits) of the block, and the sum of a 64-bit integer; `scratch` holds four of each.
+__device__ __forceinline__ uint32_t block_max_bits(uint32_t v, uint32_t *scratch)
+{
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, m, 64));
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return max(max(scratch[0], scratch[1]), max(scratch[2], scratch[3]));
+}
+__device__ __forceinline__ double block_sum_ll(long long v, long long *scratch)
+{
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return (double)(scratch[0] + scratch[1] + scratch[2] + scratch[3]);
+}
+
 // Vector-coef coefficient gradient / embedding gradient.
 //   dcoef[m] = sum_e noise(PRIME*a(e) + m) * d[e],  a(e) = e  or  idx[e / Q]*Q + e % Q.
-// grid = (ceil(k/32), splits).  A block owns 32 coefficients and the elements e = split*span .. ; its 8
-// thread groups take every 8th element of a 256-element stage buffer.  Each block writes one partial row;
-// reduce_rows_kernel adds the rows in a fixed order, so the result is reproducible.
+// A block owns a span of elements, whose digits go through LDS 256 at a time (their scale found in a pass of its own over the span),
+// and 16 MT WM coefficients, 16 MT a wave, with WM of the four waves side by side along the coefficients and 4 / WM along the
+// elements (few coefficients).  Each block writes 4 / WM partial rows; reduce_rows_kernel adds the rows in a fixed order, so the
+// result is reproducible.
 // Reference: RandumbTensor.py:304-359 (split-N + relaxed atomics there), 1059-1108.
-template <bool GATHER>
-__global__ __launch_bounds__(NT) void coef_grad_vec_kernel(float *__restrict__ partial, const void *__restrict__ d,
-                                                           int d_dtype, int64_t k, int64_t Nw, int64_t span, int64_t Q,
-                                                           uint32_t seed, const int64_t *__restrict__ idx)
+struct GradVecParams {
+    float *partial;
+    const void *d;
+    const int64_t *idx;
+    int64_t k, Nw, span, Q;
+    int d_dtype, narrow;
+    uint32_t seed;
+};
+
+template <bool GATHER> __device__ __forceinline__ uint32_t gradvec_offset(const GradVecParams &p, int64_t e)
 {
-    __shared__ float ds[NT];
-    __shared__ uint32_t as[NT];
-    __shared__ float red[8][32];
-    const int t = threadIdx.x, ml = t % 32, g = t / 32;
-    const int64_t m = (int64_t)blockIdx.x * 32 + ml;
-    const int64_t e_begin = (int64_t)blockIdx.y * span;
-    const int64_t e_end = (e_begin + span < Nw) ? e_begin + span : Nw;
-    const uint32_t mterm = (uint32_t)m * SQ5_N1 + seed;
-    float acc = 0.0f;
+    if (!GATHER) return (uint32_t)e;
+    const int64_t j = p.narrow ? (int64_t)((uint32_t)e / (uint32_t)p.Q) : e / p.Q;
+    return (uint32_t)(p.idx[j] * p.Q + (e - j * p.Q));
+}
+
+template <bool GATHER, int MT, int WM> __global__ __launch_bounds__(NT) void coef_grad_vec_kernel(GradVecParams p)
+{
+    constexpr int WE = 4 / WM, MBLOCK = 16 * MT * WM, LD = NT + 16;   // LD: eight rows apart in the banks by a quarter of them
+    __shared__ __align__(16) uint32_t win[8][LD];
+    __shared__ __align__(16) uint32_t as[NT];
+    __shared__ uint32_t tops[4];
+    __shared__ long long sums[4];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, grp = lane >> 4;
+    const int64_t e_begin = (int64_t)blockIdx.y * p.span, e_end = (e_begin + p.span < p.Nw) ? e_begin + p.span : p.Nw;
+    const int64_t m_block = (int64_t)blockIdx.x * MBLOCK, m0 = m_block + (wave % WM) * (16 * MT) + (lane & 15);
+    float *row = p.partial + ((int64_t)blockIdx.y * WE + wave / WM) * p.k;
+    uint32_t top = 0;
+    for (int64_t e = e_begin + t; e < e_end; e += NT) top = max(top, __float_as_uint(load_as_f32(p.d, p.d_dtype, e)) & 0x7fffffffu);
+    top = block_max_bits(top, tops);
+    if (top >= 0x7f800000u) {   // infinities or NaNs, which have to come out where they belong: a term at a time in fp32
+        const int64_t m_end = m_block + MBLOCK < p.k ? m_block + MBLOCK : p.k;
+        for (int64_t m = m_block + t; m < m_end; m += NT) {
+            float acc = 0.0f;
+            for (int64_t e = e_begin; e < e_end; ++e)
+                acc = fmaf(noise2d(gradvec_offset<GATHER>(p, e), (uint32_t)m, p.seed), load_as_f32(p.d, p.d_dtype, e), acc);
+            for (int r = 0; r < WE; ++r) p.partial[((int64_t)blockIdx.y * WE + r) * p.k + m] = r ? 0.0f : acc;
+        }
+        return;
+    }
+    const int ex = q8_exponent(top);
+    const double scale = pow2(ex), back = pow2(-ex) * 4.656612873077392578125e-10;
+    q8x4 acc[MT];
+    uint32_t mterm[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        acc[i] = q8x4{0, 0, 0, 0};
+        mterm[i] = (uint32_t)(m0 + i * 16) * SQ5_N1 + p.seed;
+    }
+    long long q = 0;
     for (int64_t e0 = e_begin; e0 < e_end; e0 += NT) {
-        __syncthreads();
         const int64_t e = e0 + t;
-        float dv = 0.0f;
+        float dv = 0.0f;   // zero beyond the span, so the tail adds nothing
         uint32_t a = 0;
         if (e < e_end) {
-            dv = load_as_f32(d, d_dtype, e);
-            if (GATHER) {
-                const int64_t j = e / Q;
-                a = (uint32_t)(idx[j] * Q + (e - j * Q));
-            } else {
-                a = (uint32_t)e;
+            dv = load_as_f32(p.d, p.d_dtype, e);
+            a = gradvec_offset<GATHER>(p, e);
+        }
+        uint32_t w[8];
+        q += q8_windows(dv, scale, w);
+        __syncthreads();
+        as[t] = a * PN1;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) win[s][t] = w[s];
+        __syncthreads();
+        const int steps = (int)((e_end - e0 < NT ? e_end - e0 : NT) + 15) / 16;
+        for (int st = wave / WM; st < steps; st += WE) {
+            const q8x4 d = *reinterpret_cast<const q8x4 *>(&win[lane & 7][st * 16 + grp * 4]);
+            const q8x4 f = *reinterpret_cast<const q8x4 *>(&as[st * 16 + grp * 4]);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                const q8x4 h = {q8_hash((uint32_t)f[0] + mterm[i]), q8_hash((uint32_t)f[1] + mterm[i]), q8_hash((uint32_t)f[2] + mterm[i]),
+                                q8_hash((uint32_t)f[3] + mterm[i])};
+                acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(d, h, acc[i], 0, 0, 0);
             }
         }
-        ds[t] = dv;  // zero beyond the range, so the tail adds nothing
-        as[t] = a * PN1;
-        __syncthreads();
-#pragma unroll 4
-        for (int j = 0; j < 32; ++j) {
-            const int s = j * 8 + g;
-            acc = fmaf(sq5_unit(sq5_tail(as[s] + mterm)), ds[s], acc);
-        }
     }
-    red[g][ml] = acc;
-    __syncthreads();
-    if (g == 0 && m < k) {
-        float s = red[0][ml];
+    double offset = block_sum_ll(q, sums) * Q_OFFSET;
+    if (wave / WM) offset = 0.0;   // once per block
 #pragma unroll
-        for (int j = 1; j < 8; ++j) s += red[j][ml];
-        partial[(int64_t)blockIdx.y * k + m] = s;
+    for (int i = 0; i < MT; i += 2) {   // lanes 0 .. 15: tile i, lanes 32 .. 47: tile i + 1
+        const double r = (q8_total(acc[i], acc[MT > 1 ? i + 1 : i]) + offset) * back;
+        const int64_t m = m0 + (i + (MT > 1 ? lane >> 5 : 0)) * 16;
+        if (!(grp & 1) && (MT > 1 || lane < 16) && m < p.k) row[m] = (float)r;
     }
 }
 
-// out[c] = sum_r partial[r*cols + c], rows added in index order.
-__global__ __launch_bounds__(NT) void reduce_rows_kernel(float *__restrict__ out, const float *__restrict__ partial,
-                                                         int64_t rows, int64_t cols)
+// out[c] = sum_r partial[r*cols + c] in a fixed order: 32 columns a block, 32 threads a column that take every 32nd row each (the
+// rows of a gradient's thousand blocks: one thread a column took 60 us), their sums added in thread order.
+__global__ __launch_bounds__(1024) void reduce_rows_kernel(float *__restrict__ out, const float *__restrict__ partial,
+                                                           int64_t rows, int64_t cols)
 {
-    const int64_t c = (int64_t)blockIdx.x * NT + threadIdx.x;
-    if (c >= cols) return;
+    __shared__ float part[32][33];
+    const int cl = threadIdx.x & 31, rg = threadIdx.x >> 5;
+    const int64_t c = (int64_t)blockIdx.x * 32 + cl;
     float s = 0.0f;
-    for (int64_t r = 0; r < rows; ++r) s += partial[r * cols + c];
+    if (c < cols) {
+#pragma unroll 8
+        for (int64_t r = rg; r < rows; r += 32) s += partial[r * cols + c];
+    }
+    part[rg][cl] = s;
+    __syncthreads();
+    if (rg || c >= cols) return;
+#pragma unroll
+    for (int j = 1; j < 32; ++j) s += part[j][cl];
     out[c] = s;
 }
 
@@ -283,18 +424,53 @@ __global__ __launch_bounds__(NT) void scale_bias_grad_kernel(float *__restrict__
 static inline int grid_for(int64_t n, int64_t cap = 1 << 20) { return (int)(cdiv(n, NT) < cap ? cdiv(n, NT) : cap); }
 static bool dtype_ok(int d) { return d == RDB_F32 || d == RDB_BF16; }
 
+// Coefficients a block of the gradient takes: the fewest of 16, 32, 64, 128 that hold them all (then with fewer waves along them), and
+// beyond that 64 or as many of 128 and 256 as leave no block half empty; and the partial rows a block writes.
+static int grad_block(int64_t k)
+{
+    if (k <= 32) return k <= 16 ? 16 : 32;
+    const int64_t tiles = cdiv(k, 64);
+    return tiles % 4 == 0 ? 256 : tiles % 2 == 0 ? 128 : 64;
+}
+static int grad_rows(int64_t k) { return k <= 16 ? 4 : k <= 32 ? 2 : 1; }
+
+// splits: partial rows in all
 static void split_plan(int64_t Nw, int64_t k, int64_t *splits, int64_t *span)
 {
-    // enough blocks to fill the chip (256 CUs), but spans of at least 2048 elements and a multiple of 256
-    const int64_t mblocks = cdiv(k, 32);
-    int64_t want = cdiv(2048, mblocks);
-    int64_t s = cdiv(Nw, 2048);
+    // about six blocks a compute unit (24 waves), spans of a multiple of 256 elements and of at most 2^14
+    const int64_t mblocks = cdiv(k, grad_block(k));
+    int64_t s = cdiv(Nw, NT), want = cdiv(1536, mblocks);
     if (s > want) s = want;
-    if (s < 1) s = 1;
-    int64_t sp = cdiv(cdiv(Nw, s), NT) * NT;
+    int64_t sp = cdiv(cdiv(Nw, s < 1 ? 1 : s), NT) * NT;
     if (sp < NT) sp = NT;
+    if (sp > (1 << 14)) sp = 1 << 14;
     *span = sp;
-    *splits = cdiv(Nw, sp) > 0 ? cdiv(Nw, sp) : 1;
+    *splits = (cdiv(Nw, sp) > 0 ? cdiv(Nw, sp) : 1) * grad_rows(k);
+}
+
+static int launch_materialize_vec(float *out, const void *coef, int coef_dtype, int64_t k, int64_t Nw, int64_t Q, int64_t sP, int64_t sQ, uint32_t seed,
+                                  const void *scale_bias, const int64_t *idx, hipStream_t s)
+{
+    const MatVecParams p = {out, coef, scale_bias, idx, k, Nw, Q, sP, sQ, coef_dtype, Nw < (1ll << 32) && Q < (1ll << 32), sQ == 1 && (sP == Q || Nw == Q), seed};
+    if (idx) materialize_vec_kernel<true><<<(unsigned)cdiv(Nw, NT), NT, 0, s>>>(p);
+    else materialize_vec_kernel<false><<<(unsigned)cdiv(Nw, NT), NT, 0, s>>>(p);
+    return check_launch("materialize_vec_kernel");
+}
+
+template <bool GATHER> static void launch_grad_vec(const GradVecParams &p, dim3 grid, hipStream_t s)
+{
+    switch (grad_block(p.k)) {
+    case 16: coef_grad_vec_kernel<GATHER, 1, 1><<<grid, NT, 0, s>>>(p); break;
+    case 32: coef_grad_vec_kernel<GATHER, 1, 2><<<grid, NT, 0, s>>>(p); break;
+    case 64: coef_grad_vec_kernel<GATHER, 1, 4><<<grid, NT, 0, s>>>(p); break;
+    case 128: coef_grad_vec_kernel<GATHER, 2, 4><<<grid, NT, 0, s>>>(p); break;
+    default: coef_grad_vec_kernel<GATHER, 4, 4><<<grid, NT, 0, s>>>(p); break;
+    }
+}
+static int launch_reduce_rows(float *out, const float *partial, int64_t rows, int64_t cols, hipStream_t s)
+{
+    reduce_rows_kernel<<<(unsigned)cdiv(cols, 32), 1024, 0, s>>>(out, partial, rows, cols);
+    return check_launch("reduce_rows_kernel");
 }
 
 // rdb_error.hip, rdb_f32.hip
@@ -342,9 +518,7 @@ extern "C" int rdb_materialize_fwd(float *out, const void *coef, int coef_dtype,
     if (Nw > ((int64_t)1 << 38)) return set_error(RDB_E_SHAPE, "rdb_materialize_fwd: %lld elements is too many", (long long)Nw);
     hipStream_t s = (hipStream_t)stream;
     if (coef_rows == 0) {
-        materialize_vec_kernel<false><<<(unsigned)cdiv(Nw, NT), NT, 0, s>>>(out, coef, coef_dtype, k, Nw, Q, sP, sQ, seed,
-                                                                            scale_bias, nullptr);
-        return check_launch("materialize_vec_kernel");
+        return launch_materialize_vec(out, coef, coef_dtype, k, Nw, Q, sP, sQ, seed, scale_bias, nullptr, s);
     }
     if (row_len <= 0) return set_error(RDB_E_SHAPE, "rdb_materialize_fwd: matrix-coef needs row_len > 0");
     // every addressed offset must fall inside the (coef_rows, row_len) base tensor
@@ -389,15 +563,13 @@ static int coef_grad_vec(float *dcoef, const void *d, int d_dtype, int64_t k, in
                              (long long)(splits * k * sizeof(float)), (long long)workspace_bytes);
         partial = (float *)workspace;
     }
-    dim3 grid((unsigned)cdiv(k, 32), (unsigned)splits);
-    if (idx)
-        coef_grad_vec_kernel<true><<<grid, NT, 0, s>>>(partial, d, d_dtype, k, Nw, span, Q, seed, idx);
-    else
-        coef_grad_vec_kernel<false><<<grid, NT, 0, s>>>(partial, d, d_dtype, k, Nw, span, Q, seed, nullptr);
+    const dim3 grid((unsigned)cdiv(k, grad_block(k)), (unsigned)(splits / grad_rows(k)));
+    const GradVecParams p = {partial, d, idx, k, Nw, span, Q, d_dtype, Nw < (1ll << 32) && Q < (1ll << 32), seed};
+    if (idx) launch_grad_vec<true>(p, grid, s);
+    else launch_grad_vec<false>(p, grid, s);
     int rc = check_launch("coef_grad_vec_kernel");
     if (rc || splits == 1) return rc;
-    reduce_rows_kernel<<<(unsigned)cdiv(k, NT), NT, 0, s>>>(dcoef, partial, splits, k);
-    return check_launch("reduce_rows_kernel");
+    return launch_reduce_rows(dcoef, partial, splits, k, s);
 }
 
 extern "C" int rdb_materialize_bwd(float *dcoef, const void *dW, int dw_dtype, int64_t coef_rows, int64_t k, int64_t row_len,
@@ -412,8 +584,7 @@ extern "C" int rdb_materialize_bwd(float *dcoef, const void *dW, int dw_dtype, i
     hipStream_t s = (hipStream_t)stream;
     if (coef_rows == 0) {
         if (Nw == 0) {  // empty sum
-            reduce_rows_kernel<<<(unsigned)cdiv(k, NT), NT, 0, s>>>(dcoef, dcoef, 0, k);
-            return check_launch("reduce_rows_kernel");
+            return launch_reduce_rows(dcoef, dcoef, 0, k, s);
         }
         if (!dW) return set_error(RDB_E_NULL, "rdb_materialize_bwd: dW is NULL");
         return coef_grad_vec(dcoef, dW, dw_dtype, k, Nw, 1, seed, nullptr, workspace, workspace_bytes, s, "rdb_materialize_bwd");
@@ -457,8 +628,7 @@ extern "C" int rdb_scale_bias_bwd(float *ds, const void *dW, int dw_dtype, int64
     if (!ds) return set_error(RDB_E_NULL, "rdb_scale_bias_bwd: ds is NULL");
     hipStream_t s = (hipStream_t)stream;
     if (Nw == 0) {
-        reduce_rows_kernel<<<1, NT, 0, s>>>(ds, ds, 0, 1);
-        return check_launch("reduce_rows_kernel");
+        return launch_reduce_rows(ds, ds, 0, 1, s);
     }
     if (!dW) return set_error(RDB_E_NULL, "rdb_scale_bias_bwd: dW is NULL");
     int64_t blocks, span;
@@ -473,8 +643,7 @@ extern "C" int rdb_scale_bias_bwd(float *ds, const void *dW, int dw_dtype, int64
     scale_bias_grad_kernel<<<(unsigned)blocks, NT, 0, s>>>(partial, dW, dw_dtype, Nw, span, seed);
     int rc = check_launch("scale_bias_grad_kernel");
     if (rc || blocks == 1) return rc;
-    reduce_rows_kernel<<<1, NT, 0, s>>>(ds, partial, blocks, 1);
-    return check_launch("reduce_rows_kernel");
+    return launch_reduce_rows(ds, partial, blocks, 1, s);
 }
 
 extern "C" int rdb_embed_fwd(float *out, const int64_t *idx, int64_t n_idx, const void *coef, int coef_dtype, int64_t k,
@@ -487,9 +656,7 @@ extern "C" int rdb_embed_fwd(float *out, const int64_t *idx, int64_t n_idx, cons
     const int64_t Nw = n_idx * rowsize;
     if (Nw == 0) return RDB_OK;
     if (!out || !idx || (!coef && k > 0)) return set_error(RDB_E_NULL, "rdb_embed_fwd: out, idx or coef is NULL");
-    materialize_vec_kernel<true><<<(unsigned)cdiv(Nw, NT), NT, 0, (hipStream_t)stream>>>(out, coef, coef_dtype, k, Nw, rowsize, 0,
-                                                                                         0, seed, nullptr, idx);
-    return check_launch("materialize_vec_kernel<gather>");
+    return launch_materialize_vec(out, coef, coef_dtype, k, Nw, rowsize, 0, 0, seed, nullptr, idx, (hipStream_t)stream);
 }
 
 extern "C" int64_t rdb_embed_bwd_workspace_bytes(int64_t n_idx, int64_t rowsize, int64_t k)
@@ -509,8 +676,7 @@ extern "C" int rdb_embed_bwd(float *dcoef, const int64_t *idx, int64_t n_idx, co
     hipStream_t s = (hipStream_t)stream;
     const int64_t Nw = n_idx * rowsize;
     if (Nw == 0) {
-        reduce_rows_kernel<<<(unsigned)cdiv(k, NT), NT, 0, s>>>(dcoef, dcoef, 0, k);
-        return check_launch("reduce_rows_kernel");
+        return launch_reduce_rows(dcoef, dcoef, 0, k, s);
     }
     if (!idx || !dout) return set_error(RDB_E_NULL, "rdb_embed_bwd: idx or dout is NULL");
     return coef_grad_vec(dcoef, dout, dout_dtype, k, Nw, rowsize, seed, idx, workspace, workspace_bytes, s, "rdb_embed_bwd");

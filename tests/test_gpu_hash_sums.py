@@ -1,0 +1,88 @@
+"""Vector-coef materialise, its adjoint and the embedding against fp64 sums of the noise matrix:
+sizes around the tiles' edges, views, magnitudes from denormal to huge, infinities and NaNs."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from randumb_amd import hip
+
+    return hip
+
+
+def rel(a, b):
+    return float((a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-300))
+
+
+@pytest.mark.parametrize("n,k,scale", [(1, 1, 1.0), (15, 3, 1e-3), (33, 16, 1e20), (127, 17, 1.0), (129, 64, 1e-30), (700, 65, 1.0), (1000, 256, 1e-3), (257, 1023, 1.0),
+                                       (300, 1025, 1e-42), (70, 3000, 1.0), (70001, 40, 1.0)])
+def test_sums_of_hashed_values(hip, n, k, scale):
+    print(f"case hash sums n={n} k={k} scale={scale}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    noise = hip.sq5_fill_2d(n, k, 11).double()
+    c = torch.randn(k, generator=g, device="cuda") * scale
+    d = torch.randn(n, generator=g, device="cuda") * scale
+    tol = 2e-6 if scale > 1e-38 else 0.2   # denormals have few bits themselves
+    assert rel(hip.materialize_fwd(c, (n,), (1,), 11, None, False), noise @ c.double()) < tol
+    got = hip.materialize_bwd(d, k, 11)
+    assert rel(got, d.double() @ noise) < tol
+    assert torch.equal(got, hip.materialize_bwd(d, k, 11))
+    if scale == 1.0:
+        sb = torch.tensor([0.7], device="cuda")
+        want = (noise @ c.double()) + sb.double() * hip.sq5_fill_1d(n, 11).double()
+        assert rel(hip.materialize_fwd(c, (n,), (1,), 11, sb, True), want) < tol
+        cb, db = c.bfloat16(), d.bfloat16()
+        assert rel(hip.materialize_fwd(cb, (n,), (1,), 11, None, False), noise @ cb.double()) < tol
+        assert rel(hip.materialize_bwd(db, k, 11), db.double() @ noise) < 2e-6
+
+
+def test_magnitudes_of_different_size_and_views(hip):
+    g = torch.Generator(device="cuda").manual_seed(0)
+    c = torch.randn(300, generator=g, device="cuda") * torch.exp(torch.randn(300, generator=g, device="cuda") * 4)
+    noise = hip.sq5_fill_2d(60 * 70, 300, 3).double()
+    want = (noise @ c.double()).view(60, 70)
+    assert rel(hip.materialize_fwd(c, (60, 70), (70, 1), 3, None, False), want) < 2e-6
+    assert torch.equal(hip.materialize_fwd(c, (70, 60), (1, 70), 3, None, False), hip.materialize_fwd(c, (60, 70), (70, 1), 3, None, False).t())
+    assert torch.equal(hip.materialize_fwd(c, (20, 70), (140, 1), 3, None, False), hip.materialize_fwd(c, (60, 70), (70, 1), 3, None, False)[:40:2])
+    d = torch.randn(4200, generator=g, device="cuda") * torch.exp(torch.randn(4200, generator=g, device="cuda") * 4)
+    assert rel(hip.materialize_bwd(d, 300, 3), d.double() @ noise) < 2e-6
+    one = torch.zeros(300, device="cuda")
+    one[123] = 1.0
+    assert torch.equal(hip.materialize_fwd(one, (4200,), (1,), 3, None, False), hip.sq5_fill_2d(4200, 300, 3)[:, 123])   # exact
+    assert not bool(hip.materialize_fwd(torch.zeros(300, device="cuda"), (4200,), (1,), 3, None, False).any())
+    assert not bool(hip.materialize_bwd(torch.zeros(4200, device="cuda"), 300, 3).any())
+
+
+@pytest.mark.parametrize("bad", [math.inf, -math.inf, math.nan])
+def test_infinities_and_nans_come_out(hip, bad):
+    c = torch.ones(40, device="cuda")
+    c[7] = bad
+    noise = hip.sq5_fill_2d(500, 40, 3)
+    got, want = hip.materialize_fwd(c, (500,), (1,), 3, None, False), (noise * c).sum(1)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    d = torch.ones(500, device="cuda")
+    d[300] = bad
+    got, want = hip.materialize_bwd(d, 40, 3), (noise * d[:, None]).sum(0)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+
+
+@pytest.mark.parametrize("n,dim,k", [(1, 8, 5), (9, 100, 64), (65, 33, 200), (500, 64, 300)])
+def test_embedding(hip, n, dim, k):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    idx = torch.randint(0, 50304, (n,), generator=g, device="cuda")
+    c = torch.randn(k, generator=g, device="cuda")
+    d = torch.randn(n, dim, generator=g, device="cuda")
+    table = torch.stack([_noise_rows(hip, int(i), dim, k, 9) for i in idx]).double()   # (n, dim, k)
+    assert rel(hip.embed_fwd(idx, c, dim, 9), table @ c.double()) < 2e-6
+    assert rel(hip.embed_bwd(idx, d, k, dim, 9), (d.double().unsqueeze(-1) * table).sum((0, 1))) < 2e-6
+
+
+def _noise_rows(hip, row, dim, k, seed):
+    PRIME, N1, M = 198491317, 0xD2A80A3F, 1 << 32
+    # noise(PRIME * (row * dim + r) + m, seed) = the 2-D fill's element (r, m) with the first row's offset folded into the seed
+    return hip.sq5_fill_2d(dim, k, (seed + PRIME * row * dim * N1) % M)

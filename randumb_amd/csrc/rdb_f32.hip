@@ -26,7 +26,7 @@ namespace rdb {
 
 constexpr int FG_BN = 128;        // B rows (output columns) per block
 constexpr int FG_BK = 16;         // contraction values per stage
-constexpr int FG_THREADS = 256;   // four waves, 2 x 2
+constexpr int FG_THREADS = 256;   // threads of a group: four waves, 2 x 2
 constexpr uint32_t FG_OOB = 0x80000000u;   // a byte offset past the end of any matrix these kernels take (below 2^31 bytes)
 
 // Where an operand's tile [rows x FG_BK] comes from.  In LDS every tile is [FG_BK][rows + 4]: an MFMA operand is 32
@@ -88,7 +88,7 @@ __device__ __forceinline__ void fg_split3(float v, uint32_t &h, uint32_t &m, uin
 // them into a tile.  Rows past `rows` and contraction values past `kend` are zeros.
 // VEC: the matrix is read in pieces of four values (16 bytes of fp32, 8 bytes of bf16; 16-byte aligned base, leading dimension a
 // multiple of 4, and the extent that runs along a piece a multiple of 4, so that a piece lies inside or outside as a whole);
-// otherwise value by value.
+// otherwise four values at a time at any address where all four exist, value by value at the edges.
 // SPLIT: the tile goes to LDS as three bf16 planes (see fg_split3): planes of [2 halves of the stage's 16 contraction values]
 // [rows][8] for the sources read along the contraction (a lane's MFMA operand is 16 consecutive bytes), of [16][rows + 32] for
 // FG_MCONT (read back with the LDS transpose read).  The noise sources then give a thread consecutive contraction values.
@@ -109,7 +109,8 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
     f32x4 r[NV];
 
     uint32_t inc;       // noise: first-round step per contraction value
-    int es;             // bytes per element of the matrix (2: bf16, value by value only)
+    const char *base;   // the matrix, for load4u
+    int es;             // bytes per element of the matrix (2: bf16)
     __device__ __forceinline__ float load1(uint32_t o, bool in, int j) const
     {
         if (es == 2) {
@@ -128,13 +129,27 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
         }
         return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, in ? (int)o : (int)FG_OOB, 0, 0));
     }
+    // not VEC: four consecutive elements that all exist, at any element's address (the hardware takes loads of 8 and 16 bytes at
+    // any address; 4097 tokens x 1001 features in bf16, k = 100: z = x . N^T 20.8 us with a load per value, 14.4 us with these)
+    __device__ __forceinline__ f32x4 load4u(uint32_t o) const
+    {
+        if (es == 2) {
+            typedef uint32_t pair_any __attribute__((ext_vector_type(2), aligned(2)));
+            const pair_any h = *reinterpret_cast<const pair_any *>(base + o);
+            return f32x4{__uint_as_float(h[0] << 16), __uint_as_float(h[0] & 0xffff0000u), __uint_as_float(h[1] << 16), __uint_as_float(h[1] & 0xffff0000u)};
+        }
+        typedef float quad_any __attribute__((ext_vector_type(4), aligned(4)));
+        const quad_any v = *reinterpret_cast<const quad_any *>(base + o);
+        return f32x4{v[0], v[1], v[2], v[3]};
+    }
     __device__ __forceinline__ void init(const float *src, int64_t ld, int64_t bytes, int row0, int rows, int k_begin_, int kend_, uint32_t seed,
                                          uint32_t sR, uint32_t sK, int es_)
     {
-        const int t = threadIdx.x;
+        const int t = threadIdx.x & (FG_THREADS - 1);
         k_begin = k_begin_;
         kend = kend_;
         es = es_;
+        base = reinterpret_cast<const char *>(src);
         if (SRC == FG_KCONT) {
             rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(src), 0, (int)bytes, 0x00020000);
             step = (uint32_t)(FG_BK * es);
@@ -180,6 +195,8 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
                 const uint32_t o = off[h] + (uint32_t)stage * step;
                 if (VEC) {   // all inside or all outside
                     r[h] = load4(o, ok[h] && kk < kend);
+                } else if (ok[h] && kk + 4 <= kend) {
+                    r[h] = load4u(o);
                 } else {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) r[h][j] = load1(o, ok[h] && kk + j < kend, j);
@@ -192,6 +209,8 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
                 const uint32_t o = off[h] + (uint32_t)stage * step;
                 if (VEC) {
                     r[h] = load4(o, in);
+                } else if (in && rows_left[h] >= 4) {
+                    r[h] = load4u(o);
                 } else {   // a thread's four values are consecutive rows: rows_left of them exist
 #pragma unroll
                     for (int j = 0; j < 4; ++j) r[h][j] = load1(o, in && j < rows_left[h], j);
@@ -214,7 +233,7 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
     }
     __device__ __forceinline__ void store(float *__restrict__ tile) const
     {
-        const int t = threadIdx.x;
+        const int t = threadIdx.x & (FG_THREADS - 1);
         if (SRC == FG_KCONT) {
 #pragma unroll
             for (int h = 0; h < NV; ++h) {
@@ -254,7 +273,7 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
     }
     template <bool ONE> __device__ __forceinline__ void store_split(bf16_t *__restrict__ tile) const
     {
-        const int t = threadIdx.x;
+        const int t = threadIdx.x & (FG_THREADS - 1);
         if (SRC == FG_KCONT) {
 #pragma unroll
             for (int h = 0; h < NV; ++h) {   // contraction values 4 kq .. 4 kq + 3 of a row
@@ -292,20 +311,35 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
     }
 };
 
-// out[M x N] (+)= A . B^T over one split of the contraction.  Block: BM x 128 of the output, four waves as 2 x 2, a wave owns
-// (BM / 2) x 64 in BM / 64 x 2 accumulator tiles.  Two LDS buffers, one barrier per stage: while a stage is multiplied the
-// next one is on its way from memory (or being hashed) in registers.
-template <int BM, int ASRC, int BSRC, int EPI, bool VEC, bool SPLIT = false, bool ANY16 = false>
-__global__ __launch_bounds__(FG_THREADS, 2) void f32_gemm_kernel(FgParams p)
+// out[M x N] (+)= A . B^T over one split of the contraction.  Block: BM x 128 of the output, G groups of four waves as 2 x 2, a
+// wave owns (BM / 2) x 64 in BM / 64 x 2 accumulator tiles.  Two LDS buffers, one barrier per stage: while a stage is multiplied
+// the next one is on its way from memory (or being hashed) in registers.
+// G groups cut the block's contraction into G runs of stages, each with its own LDS buffers, and add their accumulators up
+// through LDS in group order at the end.  One group is one wave to a SIMD, and its stages are a serial chain of about 1 us (load,
+// split, barrier, LDS read, products, hash): a product with fewer blocks than compute units is bound by that chain, and G of
+// them run side by side.  2048 tokens x 768 -> 3072, k = 256, fp32: z = x . N^T 14.6 us (64 rows, 6 ranges) -> 10.3 (G = 4, 4
+// ranges), dx = t . N 19.5 -> 11.7 (G = 4), t = dy . C 27.4 us in 16 ranges -> 23.4 in 8 (G = 2: half the partial sums).  With
+// blocks enough the chip's power is the bound (1.75 GHz under y = z . C^T, 3 groups a unit), and how the groups are arranged
+// matters little.
+// Results leave with streaming stores: they would be written back from L2 at the end of the kernel otherwise, after the last
+// block (y of that layer, 25 MB: 26.4 -> 24.8 us).
+template <int BM, int G, int ASRC, int BSRC, int EPI, bool VEC, bool SPLIT = false, bool ANY16 = false>
+__global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kernel(FgParams p)
 {
     typedef FgOperand<BM, ASRC, VEC, SPLIT> PA;
     typedef FgOperand<FG_BN, BSRC, VEC, SPLIT> PB;
     constexpr int MI = BM / 64, NI = 2, STAGE = (PA::TILE_BYTES + PB::TILE_BYTES) / 4;   // floats
-    __shared__ __align__(16) float lds[2 * STAGE];
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, r = lane & 31, g = lane >> 5, wm = wave >> 1, wn = wave & 1;
+    static_assert(G == 1 || SPLIT, "groups: the bf16 matrix instructions only");
+    constexpr int UNITS = MI * NI * 2;   // a wave's accumulators in units of 8 registers: what the groups share out at the end
+    constexpr int EXCHANGE = (G - 1) * UNITS * 4 * 512;
+    __shared__ __align__(16) float lds_all[2 * STAGE * G > EXCHANGE ? 2 * STAGE * G : EXCHANGE];
+    const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / FG_THREADS);
+    float *lds = lds_all + group * 2 * STAGE;
+    const int t = threadIdx.x & (FG_THREADS - 1), wave = t >> 6, lane = t & 63, r = lane & 31, g = lane >> 5, wm = wave >> 1, wn = wave & 1;
     const int m0 = blockIdx.x * BM, n0 = blockIdx.y * FG_BN;   // the long extent (tokens, as a rule) on the grid's x
-    const int k_begin = blockIdx.z * p.kchunk, kend = min(p.K, k_begin + p.kchunk);
-    const int nstage = (kend - k_begin + FG_BK - 1) / FG_BK;
+    const int k_first = blockIdx.z * p.kchunk, k_last = min(p.K, k_first + p.kchunk);
+    const int nstage = ((k_last - k_first + FG_BK - 1) / FG_BK + G - 1) / G;   // of every group: the last one's may be empty
+    const int k_begin = k_first + group * nstage * FG_BK, kend = min(k_last, k_begin + nstage * FG_BK);
     PA pa;
     PB pb;
     pa.init(p.a, p.lda, p.a_bytes, m0, p.M, k_begin, kend, p.seed, p.nsR, p.nsK, p.a_es);
@@ -421,6 +455,32 @@ __global__ __launch_bounds__(FG_THREADS, 2) void f32_gemm_kernel(FgParams p)
             else stages(One{}, One{});
         }
     }
+    if constexpr (G > 1) {
+        // unit u (registers 8 (u % 2) .. of tile u / 2) is finished by group u * G / UNITS; the others hand theirs over
+        __syncthreads();   // the stage buffers are free
+        auto slot = [&](int u, int from, int owner) { return lds_all + ((u * (G - 1) + (from < owner ? from : from - 1)) * 4 + wave) * 512 + lane; };
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u) {
+            const int owner = u * G / UNITS;
+            if (group == owner) continue;
+            float *dst = slot(u, group, owner);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) dst[j * 64] = acc[u / 2 / NI][u / 2 % NI][(u & 1) * 8 + j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u) {
+            const int owner = u * G / UNITS;
+            if (group != owner) continue;
+#pragma unroll
+            for (int from = 0; from < G; ++from) {
+                if (from == owner) continue;
+                const float *src = slot(u, from, owner);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc[u / 2 / NI][u / 2 % NI][(u & 1) * 8 + j] += src[j * 64];
+            }
+        }
+    }
     // accumulator j of lane (r, g): row 8 (j / 4) + 4 g + j % 4 of the A side, column r of the B side
     float *out = p.out + (int64_t)blockIdx.z * p.split_stride;
     bf16_t *out16 = reinterpret_cast<bf16_t *>(p.out);   // bf16 outputs are never the ranges' partial matrices
@@ -437,6 +497,7 @@ __global__ __launch_bounds__(FG_THREADS, 2) void f32_gemm_kernel(FgParams p)
         for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
+                if (G > 1 && group != ((mi * NI + ni) * 2 + j / 8) * G / UNITS) continue;
                 const int m = m0 + wm * (BM / 2) + mi * 32 + 8 * (j >> 2) + 4 * g + (j & 3);
                 if (m >= p.M) continue;
                 const float a = acc[mi][ni][j];
@@ -447,7 +508,8 @@ __global__ __launch_bounds__(FG_THREADS, 2) void f32_gemm_kernel(FgParams p)
                     const int64_t e = (int64_t)m * p.ldo + n;
                     if (EPI == FG_STORE_RBIAS) out[e] = fmaf(scale, noise1d((uint32_t)m * p.nsR + (uint32_t)n * p.nsK, p.seed), a);
                     else if (o16) out16[e] = f32_to_bf16(EPI == FG_ADD_SCALED ? fmaf(scale, a, bf16_to_f32(out16[e])) : a + bv);
-                    else out[e] = EPI == FG_ADD_SCALED ? fmaf(scale, a, out[e]) : a + bv;
+                    else if (EPI == FG_ADD_SCALED) out[e] = fmaf(scale, a, out[e]);
+                    else __builtin_nontemporal_store(a + bv, out + e);
                 }
             }
     }
@@ -478,19 +540,22 @@ __global__ __launch_bounds__(256) void f32_sum_scalars_kernel(float *__restrict_
 }
 
 // out[i] = part[0][i] + part[1][i] + ... in split order, four values per thread (n4 groups of four, then the n % 4 last values
-// one thread each)
-__global__ __launch_bounds__(256) void f32_sum_splits_kernel(float *__restrict__ out, const float *__restrict__ part, int64_t n, int64_t stride, int splits, int vec)
+// one thread each); out fp32, or bf16 (rounded once)
+__global__ __launch_bounds__(256) void f32_sum_splits_kernel(void *__restrict__ out, int out_bf16, const float *__restrict__ part, int64_t n, int64_t stride,
+                                                             int splits, int vec)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, n4 = vec ? n / 4 : 0;
     if (i < n4) {
         f32x4 v = *reinterpret_cast<const f32x4 *>(part + i * 4);
         for (int s = 1; s < splits; ++s) v += *reinterpret_cast<const f32x4 *>(part + s * stride + i * 4);
-        *reinterpret_cast<f32x4 *>(out + i * 4) = v;
+        if (out_bf16) store4<bf16_t>(static_cast<bf16_t *>(out) + i * 4, v[0], v[1], v[2], v[3]);
+        else *reinterpret_cast<f32x4 *>(static_cast<float *>(out) + i * 4) = v;
     } else if (n4 * 4 + (i - n4) < n) {
         const int64_t e = n4 * 4 + (i - n4);
         float v = part[e];
         for (int s = 1; s < splits; ++s) v += part[s * stride + e];
-        out[e] = v;
+        if (out_bf16) static_cast<bf16_t *>(out)[e] = f32_to_bf16(v);
+        else static_cast<float *>(out)[e] = v;
     }
 }
 
@@ -511,15 +576,26 @@ static int fg_es(int dtype) { return dtype == RDB_BF16 ? 2 : 4; }
 // few TFLOP/s, so the factored form on the matrix cores wins also where it is more flops than a product on a stored W.
 static bool fg_wanted(const rdb_linear_desc *) { return true; }
 
-// Tile height and number of contraction ranges of a product [M x N] over K.  Planned for two blocks per compute unit at a
-// time (the hardware takes up to four).  A product with fewer tiles than that is cut into ranges of the contraction (at least
-// min_range values each, at most max_ranges): each range leaves a partial matrix, added up in range order afterwards, so the
-// result does not depend on which block finishes first.  128-row tiles unless even in ranges they would leave half of the
-// compute units without a block; 64-row tiles then.
+// 1 (default): the linear layers' products run as six bf16 matrix instructions on three-way splits of their operands
+// (fg_split3); 0: as fp32 matrix instructions.  Process-wide (rdb_set_f32_split).
+static int g_f32_split = 1;
+int f32_split_mode() { return g_f32_split; }
+int set_f32_split_mode(int mode)
+{
+    const int old = g_f32_split;
+    g_f32_split = mode ? 1 : 0;
+    return old;
+}
+
+// How a product [M x N] over K runs: tile height, groups per block, contraction ranges.  Each range leaves a partial matrix,
+// added up in range order afterwards, so the result does not depend on which block finishes first.
 struct FgPlan {
-    int bm, ranges;
+    int bm, ranges, groups;
 };
-static FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int64_t min_range, int max_ranges)
+// Room for partial matrices: what a workspace holds.  128-row tiles, two blocks per compute unit at a time, unless even in ranges
+// they would leave half of the compute units without a block; 64-row tiles then.  A product with fewer tiles than that is cut
+// into ranges of the contraction, at least min_range values each, at most max_ranges.
+static FgPlan fg_room(int64_t M, int64_t N, int64_t K, int num_cus, int64_t min_range, int max_ranges)
 {
     const int64_t slots = 2 * (int64_t)num_cus;
     const int64_t t128 = cdiv(M, 128) * cdiv(N, FG_BN), t64 = cdiv(M, 64) * cdiv(N, FG_BN);
@@ -532,12 +608,48 @@ static FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int64_t min_
         return r < 1 ? (int64_t)1 : r;
     };
     const int64_t r128 = ranges(t128), r64 = ranges(t64);
-    if (t128 * r128 * 2 < slots) return {64, (int)r64};
-    return {128, (int)r128};
+    if (t128 * r128 * 2 < slots) return {64, (int)r64, 1};
+    return {128, (int)r128, 1};
 }
-// z = x . N^T and t = dy . C, [tokens x k] over K = in_f or out_f; dC = dy^T . z, [out_f x k] over the tokens
-static FgPlan zt_plan(const rdb_linear_desc *d, int64_t K, int num_cus) { return fg_plan(d->tokens, d->k, K, num_cus, 128, 32); }
-static FgPlan dc_plan(const rdb_linear_desc *d, int num_cus) { return fg_plan(d->out_f, d->k, d->tokens, num_cus, 256, 64); }
+// The plan with the least modelled time, of those with at most max_ranges ranges.  The model is measured (22 products of this
+// file's kinds, [258 .. 7520] x [100 .. 7520] over [100 .. 7520], some 380 plans; what it picks is within 1 % of the best of
+// them on average, 3 % at most): a stage of a group takes `chain` us when it has the compute unit to itself, the groups that
+// share a unit take `unit` us of its throughput each, a launch `base` us and every further round of blocks 2.6; outputs leave at 4.8 TB/s; adding ranges up is one more
+// launch, whose 14 TB/s say that the partial matrices come back out of the caches.  Blocks that run on a unit at a time: what
+// registers and LDS leave room for.
+static FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int max_ranges, bool groups4)
+{
+    struct Kind {
+        int bm, groups, resident;
+        double chain, unit, base;
+    };
+    static const Kind kinds[] = {{128, 1, 3, 0.51, 0.36, 5.4}, {128, 2, 1, 0.51, 0.36, 5.4}, {64, 1, 4, 0.46, 0.26, 3.7},
+                                 {64, 2, 2, 0.46, 0.26, 3.7},  {64, 4, 1, 0.46, 0.26, 3.7}};
+    const bool split = f32_split_mode() != 0;
+    const double out_mb = (double)M * N * 4e-6;
+    FgPlan best = {128, 1, 1};
+    double best_us = 1e30;
+    for (const Kind &kd : kinds) {
+        if (kd.groups > 1 && (!split || (kd.groups == 4 && !groups4))) continue;
+        const int64_t tiles = cdiv(M, kd.bm) * cdiv(N, FG_BN);
+        for (int r = 1; r <= max_ranges; ++r) {
+            const int64_t chunk = cdiv(cdiv(K, r), FG_BK) * FG_BK;
+            if (r > 1 && (cdiv(K, chunk) != r || chunk < 64)) continue;   // every range holds something, and four stages at least
+            const int64_t per_cu = cdiv(tiles * r, num_cus), stages = cdiv(chunk / FG_BK, kd.groups);
+            const int64_t rounds = cdiv(per_cu, kd.resident);
+            const double us = kd.base + 2.6 * (rounds - 1) + stages * (rounds * kd.chain + per_cu * kd.groups * kd.unit) + out_mb * r * 0.21 +
+                              (r > 1 ? 4.2 + out_mb * r * 0.07 : 0.0);
+            if (us < best_us) {
+                best_us = us;
+                best = {kd.bm, r, kd.groups};
+            }
+        }
+    }
+    return best;
+}
+// z = x . N^T and t = dy . C, [tokens x k] over K = in_f or out_f; dC = dy^T . z, [out_f x k] over the tokens: ranges there is room for
+static int zt_room(const rdb_linear_desc *d, int64_t K, int num_cus) { return fg_room(d->tokens, d->k, K, num_cus, 128, 32).ranges; }
+static int dc_room(const rdb_linear_desc *d, int num_cus) { return fg_room(d->out_f, d->k, d->tokens, num_cus, 256, 64).ranges; }
 
 // scratch: z or t [tokens x k] and its partial matrices; for the coefficient gradient also one [out_f x k] matrix per token range
 int64_t linear_f32_workspace(int op, const rdb_linear_desc *d, int num_cus)
@@ -546,24 +658,13 @@ int64_t linear_f32_workspace(int op, const rdb_linear_desc *d, int num_cus)
     if (op == RDB_OP_LINEAR_BWD_DCOEF) dd.coef_dtype = dd.act_dtype;   // reads no coefficients
     if (!fg_ok(&dd)) return 0;
     const int64_t zt = up256(d->tokens * d->k * 4);
-    auto with_parts = [&](int64_t K) { const int r = zt_plan(d, K, num_cus).ranges; return zt * (r > 1 ? 1 + r : 1); };
+    auto with_parts = [&](int64_t K) { const int r = zt_room(d, K, num_cus); return zt * (r > 1 ? 1 + r : 1); };
     if (op == RDB_OP_LINEAR_FWD) return with_parts(d->in_f);
     if (op == RDB_OP_LINEAR_BWD_DX) return with_parts(d->out_f);
     if (op != RDB_OP_LINEAR_BWD_DCOEF) return 0;
-    const int r = dc_plan(d, num_cus).ranges;
+    const int r = dc_room(d, num_cus);
     // ... and, for the gradient of the random bias's scale, one value per 64 x 128 tile of [tokens x out_f]
     return with_parts(d->in_f) + (r > 1 ? (int64_t)r * up256(d->out_f * d->k * 4) : 0) + up256(cdiv(d->tokens, 64) * cdiv(d->out_f, FG_BN) * 4);
-}
-
-// 1 (default): the linear layers' products run as six bf16 matrix instructions on three-way splits of their operands
-// (fg_split3); 0: as fp32 matrix instructions.  Process-wide (rdb_set_f32_split).
-static int g_f32_split = 1;
-int f32_split_mode() { return g_f32_split; }
-int set_f32_split_mode(int mode)
-{
-    const int old = g_f32_split;
-    g_f32_split = mode ? 1 : 0;
-    return old;
 }
 
 struct FgProduct {
@@ -575,7 +676,8 @@ struct FgProduct {
     int64_t ldo;
     const float *bias;
     int64_t M, N, K;
-    int bm;                 // tile height: 128 or 64
+    int bm;                 // tile height: 128 or 64; 0: fg_launch plans it, and the groups
+    int groups;             // per block: 1, 2 or (64-row tiles) 4
     int64_t kchunk;         // contraction values per range (a multiple of FG_BK); 0: one range
     int64_t split_stride;   // floats between the ranges' outputs
     uint32_t seed;
@@ -592,19 +694,37 @@ struct FgProduct {
     bool split = f32_split_mode() != 0;
 };
 
-#define FG_LAUNCH(BM_, EPI_)                                                                                  \
-    do {                                                                                                      \
-        if (q.split && any16) {                                                                               \
-            if (vec) f32_gemm_kernel<BM_, ASRC, BSRC, EPI_, true, true, true><<<grid, FG_THREADS, 0, s>>>(p); \
-            else f32_gemm_kernel<BM_, ASRC, BSRC, EPI_, false, true, true><<<grid, FG_THREADS, 0, s>>>(p);    \
-        } else if (q.split) {                                                                                 \
-            if (vec) f32_gemm_kernel<BM_, ASRC, BSRC, EPI_, true, true><<<grid, FG_THREADS, 0, s>>>(p);       \
-            else f32_gemm_kernel<BM_, ASRC, BSRC, EPI_, false, true><<<grid, FG_THREADS, 0, s>>>(p);          \
-        } else if (vec) f32_gemm_kernel<BM_, ASRC, BSRC, EPI_, true><<<grid, FG_THREADS, 0, s>>>(p);          \
-        else f32_gemm_kernel<BM_, ASRC, BSRC, EPI_, false><<<grid, FG_THREADS, 0, s>>>(p);                    \
+#define FG_LAUNCH_GROUPS(BM_, G_, EPI_)                                                                               \
+    do {                                                                                                            \
+        const int nt = FG_THREADS * G_;                                                                             \
+        if (any16) {                                                                                                \
+            if (vec) f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, true, true, true><<<grid, nt, 0, s>>>(p);           \
+            else f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, false, true, true><<<grid, nt, 0, s>>>(p);              \
+        } else {                                                                                                    \
+            if (vec) f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, true, true><<<grid, nt, 0, s>>>(p);                 \
+            else f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, false, true><<<grid, nt, 0, s>>>(p);                    \
+        }                                                                                                           \
     } while (0)
-template <int ASRC, int BSRC> static int fg_launch(const FgProduct &q, int num_cus, hipStream_t s, const char *name)
+#define FG_LAUNCH(BM_, EPI_)                                                                                        \
+    do {                                                                                                            \
+        if (q.split) FG_LAUNCH_GROUPS(BM_, 1, EPI_);                                                                \
+        else if (vec) f32_gemm_kernel<BM_, 1, ASRC, BSRC, EPI_, true><<<grid, FG_THREADS, 0, s>>>(p);               \
+        else f32_gemm_kernel<BM_, 1, ASRC, BSRC, EPI_, false><<<grid, FG_THREADS, 0, s>>>(p);                       \
+    } while (0)
+// The kernels with several groups per block, and whether there is one: four groups' buffers do not fit in LDS where a side is read
+// across its rows (its planes are padded), and only the plain epilogues are built.
+template <int ASRC, int BSRC> struct FgGroups {
+    static constexpr bool any = BSRC != FG_NOISE_1D, four = any && ASRC != FG_MCONT && BSRC != FG_MCONT;
+};
+template <int ASRC, int BSRC> static int fg_launch(FgProduct q, int num_cus, hipStream_t s, const char *name)
 {
+    typedef FgGroups<ASRC, BSRC> Groups;
+    if (!q.bm) {
+        const bool plain = Groups::any && !q.scale;
+        const FgPlan pl = plain ? fg_plan(q.M, q.N, q.K, num_cus, 1, Groups::four) : fg_room(q.M, q.N, q.K, num_cus, q.K, 1);
+        q.bm = pl.bm;
+        q.groups = pl.groups;
+    }
     if (q.a_elems >= (1ll << 29) || q.b_elems >= (1ll << 29) || q.M >= (1ll << 30) || q.N >= (1ll << 30) || q.K >= (1ll << 30)) return RDB_E_UNSUPPORTED;
     FgParams p = {};
     p.a = q.a;
@@ -643,7 +763,7 @@ template <int ASRC, int BSRC> static int fg_launch(const FgProduct &q, int num_c
     const bool any16 = q.a_es == 2 || ((BSRC == FG_KCONT || BSRC == FG_MCONT) && q.b_es == 2);   // the A side is always a matrix
     if (cdiv(q.N, FG_BN) > 65535) return RDB_E_UNSUPPORTED;   // the grid's y
     const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)splits);
-    if (BSRC == FG_NOISE_1D) {   // the random-bias products: added on top of an output, or reduced against a matrix
+    if constexpr (BSRC == FG_NOISE_1D) {   // the random-bias products: added on top of an output, or reduced against a matrix
         if (q.bm == 128) {
             if (q.dotm) FG_LAUNCH(128, FG_DOT);
             else FG_LAUNCH(128, FG_ADD_SCALED);
@@ -654,9 +774,20 @@ template <int ASRC, int BSRC> static int fg_launch(const FgProduct &q, int num_c
     } else if (q.scale) {        // materialising W with its random-bias share
         if (q.bm == 128) FG_LAUNCH(128, FG_STORE_RBIAS);
         else FG_LAUNCH(64, FG_STORE_RBIAS);
+    } else if (q.bm == 128 && q.groups == 2) {
+        if (q.bias) FG_LAUNCH_GROUPS(128, 2, FG_STORE_BIAS);
+        else FG_LAUNCH_GROUPS(128, 2, FG_STORE);
     } else if (q.bm == 128) {
         if (q.bias) FG_LAUNCH(128, FG_STORE_BIAS);
         else FG_LAUNCH(128, FG_STORE);
+    } else if (q.groups == 2) {
+        if (q.bias) FG_LAUNCH_GROUPS(64, 2, FG_STORE_BIAS);
+        else FG_LAUNCH_GROUPS(64, 2, FG_STORE);
+    } else if (q.groups == 4) {
+        if constexpr (Groups::four) {
+            if (q.bias) FG_LAUNCH_GROUPS(64, 4, FG_STORE_BIAS);
+            else FG_LAUNCH_GROUPS(64, 4, FG_STORE);
+        }
     } else {
         if (q.bias) FG_LAUNCH(64, FG_STORE_BIAS);
         else FG_LAUNCH(64, FG_STORE);
@@ -669,45 +800,38 @@ static bool fg_ws_ok(int op, const rdb_linear_desc *d, int num_cus, const void *
     return ws && fg_aligned16(ws) && bytes >= linear_f32_workspace(op, d, num_cus);
 }
 
-static int fg_sum(float *out, const float *part, int64_t n, int64_t stride, int splits, hipStream_t s)
+// A product whose dense output [M x N] (ldo = N) may be computed in up to `room` ranges of the contraction: the ranges' partial
+// matrices go to `part` (stride floats apart) and are added up into q.out in range order.
+template <int ASRC, int BSRC> static int fg_launch_ranges(FgProduct q, int room, float *part, int64_t stride, int num_cus, hipStream_t s, const char *name)
 {
+    const FgPlan plan = fg_plan(q.M, q.N, q.K, num_cus, room, FgGroups<ASRC, BSRC>::four);
+    q.bm = plan.bm;
+    q.groups = plan.groups;
+    q.kchunk = 0;
+    q.split_stride = 0;
+    if (plan.ranges <= 1) return fg_launch<ASRC, BSRC>(q, num_cus, s, name);
+    float *const out = q.out;
+    const int out_bf16 = q.out_bf16;
+    const int64_t n = q.M * q.N;
+    q.out = part;
+    q.out_bf16 = 0;
+    q.kchunk = cdiv(cdiv(q.K, plan.ranges), FG_BK) * FG_BK;   // every range holds something (fg_plan)
+    q.split_stride = stride;
+    if (int rc = fg_launch<ASRC, BSRC>(q, num_cus, s, name)) return rc;
     const int vec = fg_aligned16(out) ? 1 : 0;   // the partial matrices are 256-byte aligned
-    f32_sum_splits_kernel<<<(unsigned)cdiv(vec ? n / 4 + n % 4 : n, 256), 256, 0, s>>>(out, part, n, stride, splits, vec);
+    f32_sum_splits_kernel<<<(unsigned)cdiv(vec ? n / 4 + n % 4 : n, 256), 256, 0, s>>>(out, out_bf16, part, n, stride, plan.ranges, vec);
     return check_launch("f32_sum_splits_kernel");
 }
 
-// A product whose dense output [M x N] (ldo = N) may be computed in `splits` ranges of the contraction: the ranges' partial
-// matrices go to `part` (stride floats apart) and are added up into q.out in range order.
-template <int ASRC, int BSRC> static int fg_launch_ranges(FgProduct q, FgPlan plan, float *part, int64_t stride, int num_cus, hipStream_t s, const char *name)
-{
-    int splits = plan.ranges;
-    q.bm = plan.bm;
-    const int kchunk = (int)(cdiv(cdiv(q.K, splits), FG_BK) * FG_BK);
-    splits = (int)cdiv(q.K, kchunk);   // the ranges that hold something
-    if (splits <= 1) {
-        q.kchunk = 0;
-        q.split_stride = 0;
-        return fg_launch<ASRC, BSRC>(q, num_cus, s, name);
-    }
-    float *out = q.out;
-    q.out = part;
-    q.kchunk = kchunk;
-    q.split_stride = stride;
-    if (int rc = fg_launch<ASRC, BSRC>(q, num_cus, s, name)) return rc;
-    return fg_sum(out, part, q.M * q.N, stride, splits, s);
-}
-
 // z[T x k] = src[T x in_f] . N^T; the partial matrices of its ranges go to `part` (room for max_ranges of them, up256(T k 4)
-// bytes apart; NULL: right behind z, as many as the plan wants)
+// bytes apart; NULL: right behind z, as many as there is room for)
 static int fg_project(float *z, const float *x, int64_t ldx, const rdb_linear_desc *d, int num_cus, hipStream_t s, float *part = nullptr,
                       int max_ranges = 1 << 30)
 {
-    FgProduct q = {x, ldx, (d->tokens - 1) * ldx + d->in_f, nullptr, 0, 0, z, d->k, nullptr, d->tokens, d->k, d->in_f, 128, 0, 0, d->seed};
+    FgProduct q = {x, ldx, (d->tokens - 1) * ldx + d->in_f, nullptr, 0, 0, z, d->k, nullptr, d->tokens, d->k, d->in_f, 0, 0, 0, 0, d->seed};
     q.a_es = fg_es(d->act_dtype);
     const int64_t zt = up256(d->tokens * d->k * 4) / 4;
-    FgPlan plan = zt_plan(d, d->in_f, num_cus);
-    if (plan.ranges > max_ranges) plan.ranges = max_ranges < 1 ? 1 : max_ranges;
-    return fg_launch_ranges<FG_KCONT, FG_NOISE_M>(q, plan, part ? part : z + zt, zt, num_cus, s, "f32_gemm_kernel (z = x . N^T)");
+    return fg_launch_ranges<FG_KCONT, FG_NOISE_M>(q, std::max(1, std::min(zt_room(d, d->in_f, num_cus), max_ranges)), part ? part : z + zt, zt, num_cus, s, "f32_gemm_kernel (z = x . N^T)");
 }
 
 // The three entry points return RDB_E_UNSUPPORTED, without setting an error, when the request does not fit.
@@ -719,7 +843,7 @@ int linear_fwd_f32(void *y, int64_t ldy, const void *x, int64_t ldx, const void 
     float *z = (float *)workspace;
     if (int rc = fg_project(z, (const float *)x, ldx, d, num_cus, s)) return rc;
     FgProduct q = {z, d->k, d->tokens * d->k, (const float *)coef, d->k, d->out_f * d->k, (float *)y, ldy, (const float *)bias,
-                   d->tokens, d->out_f, d->k, fg_plan(d->tokens, d->out_f, d->k, num_cus, d->k, 1).bm, 0, 0, d->seed};
+                   d->tokens, d->out_f, d->k, 0, 0, 0, 0, d->seed};
     const int b16 = d->act_dtype == RDB_BF16;
     q.b_es = fg_es(d->coef_dtype);
     q.out_bf16 = b16;
@@ -727,7 +851,7 @@ int linear_fwd_f32(void *y, int64_t ldy, const void *x, int64_t ldx, const void 
     if (!scale_bias) return RDB_OK;
     // y += s * x . R^T: the B side's rows are output features, index o * in_f + i
     FgProduct qr = {(const float *)x, ldx, (d->tokens - 1) * ldx + d->in_f, nullptr, 0, 0, (float *)y, ldy, nullptr, d->tokens, d->out_f, d->in_f,
-                    fg_plan(d->tokens, d->out_f, d->in_f, num_cus, d->in_f, 1).bm, 0, 0, d->seed, (uint32_t)d->in_f, 1u, (const float *)scale_bias,
+                    0, 0, 0, 0, d->seed, (uint32_t)d->in_f, 1u, (const float *)scale_bias,
                     nullptr, 0, nullptr};
     qr.a_es = fg_es(d->act_dtype);
     qr.out_bf16 = b16;
@@ -743,21 +867,21 @@ int linear_dx_f32(void *dx, int64_t lddx, const void *dy, int64_t lddy, const vo
     float *t = (float *)workspace;
     // t[T x k] = dy[T x out_f] . C: the B side's rows are coefficients, read across the rows of C
     FgProduct q1 = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, (const float *)coef, d->k, d->out_f * d->k, t, d->k, nullptr,
-                    d->tokens, d->k, d->out_f, 128, 0, 0, d->seed};
+                    d->tokens, d->k, d->out_f, 0, 0, 0, 0, d->seed};
     const int b16 = d->act_dtype == RDB_BF16;
     q1.a_es = fg_es(d->act_dtype);
     q1.b_es = fg_es(d->coef_dtype);
     const int64_t zt = up256(d->tokens * d->k * 4) / 4;
-    if (int rc = fg_launch_ranges<FG_KCONT, FG_MCONT>(q1, zt_plan(d, d->out_f, num_cus), t + zt, zt, num_cus, s, "f32_gemm_kernel (t = dy . C)")) return rc;
+    if (int rc = fg_launch_ranges<FG_KCONT, FG_MCONT>(q1, zt_room(d, d->out_f, num_cus), t + zt, zt, num_cus, s, "f32_gemm_kernel (t = dy . C)")) return rc;
     // dx[T x in_f] = t . N: the B side's rows are input features, hashed
     FgProduct q2 = {t, d->k, d->tokens * d->k, nullptr, 0, 0, (float *)dx, lddx, nullptr, d->tokens, d->in_f, d->k,
-                    fg_plan(d->tokens, d->in_f, d->k, num_cus, d->k, 1).bm, 0, 0, d->seed};
+                    0, 0, 0, 0, d->seed};
     q2.out_bf16 = b16;
     if (int rc = fg_launch<FG_KCONT, FG_NOISE_I>(q2, num_cus, s, "f32_gemm_kernel (dx = t . N)")) return rc;
     if (!scale_bias) return RDB_OK;
     // dx += s * dy . R: the B side's rows are input features, index o * in_f + i
     FgProduct qr = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, nullptr, 0, 0, (float *)dx, lddx, nullptr, d->tokens, d->in_f, d->out_f,
-                    fg_plan(d->tokens, d->in_f, d->out_f, num_cus, d->out_f, 1).bm, 0, 0, d->seed, 1u, (uint32_t)d->in_f, (const float *)scale_bias,
+                    0, 0, 0, 0, d->seed, 1u, (uint32_t)d->in_f, (const float *)scale_bias,
                     nullptr, 0, nullptr};
     qr.a_es = fg_es(d->act_dtype);
     qr.out_bf16 = b16;
@@ -777,18 +901,18 @@ int linear_dcoef_f32(float *dcoef, float *d_scale_bias, const void *dy, int64_t 
     float *z = (float *)workspace;
     if (int rc = fg_project(z, (const float *)x, ldx, &dd, num_cus, s)) return rc;
     // dC[out_f x k] = dy^T . z: both sides are read across their rows (the contraction runs over the tokens)
-    const int zs = zt_plan(&dd, d->in_f, num_cus).ranges;
+    const int zs = zt_room(&dd, d->in_f, num_cus);
     float *part = reinterpret_cast<float *>(static_cast<char *>(workspace) + up256(d->tokens * d->k * 4) * (zs > 1 ? 1 + zs : 1));
     FgProduct q = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, z, d->k, d->tokens * d->k, dcoef, d->k, nullptr,
-                   d->out_f, d->k, d->tokens, 128, 0, 0, d->seed};
-    const FgPlan dcp = dc_plan(&dd, num_cus);
+                   d->out_f, d->k, d->tokens, 0, 0, 0, 0, d->seed};
+    const int dcr = dc_room(&dd, num_cus);
     q.a_es = fg_es(d->act_dtype);
-    if (int rc = fg_launch_ranges<FG_MCONT, FG_MCONT>(q, dcp, part, up256(d->out_f * d->k * 4) / 4, num_cus, s, "f32_gemm_kernel (dC = dy^T . z)")) return rc;
+    if (int rc = fg_launch_ranges<FG_MCONT, FG_MCONT>(q, dcr, part, up256(d->out_f * d->k * 4) / 4, num_cus, s, "f32_gemm_kernel (dC = dy^T . z)")) return rc;
     if (!d_scale_bias) return RDB_OK;
     // <dy, x . R^T>: the random-bias product once more, each block reducing its tile against dy's; then the blocks in order
-    float *dots = part + (dcp.ranges > 1 ? (int64_t)dcp.ranges * (up256(d->out_f * d->k * 4) / 4) : 0);
+    float *dots = part + (dcr > 1 ? (int64_t)dcr * (up256(d->out_f * d->k * 4) / 4) : 0);
     FgProduct qr = {(const float *)x, ldx, (d->tokens - 1) * ldx + d->in_f, nullptr, 0, 0, nullptr, 0, nullptr, d->tokens, d->out_f, d->in_f,
-                    fg_plan(d->tokens, d->out_f, d->in_f, num_cus, d->in_f, 1).bm, 0, 0, d->seed, (uint32_t)d->in_f, 1u, nullptr,
+                    fg_room(d->tokens, d->out_f, d->in_f, num_cus, d->in_f, 1).bm, 1, 0, 0, d->seed, (uint32_t)d->in_f, 1u, nullptr,
                     (const float *)dy, lddy, dots};
     qr.a_es = fg_es(d->act_dtype);
     qr.out_bf16 = d->act_dtype == RDB_BF16;   // dy, the matrix the product is reduced against
@@ -803,21 +927,21 @@ int linear_dcoef_f32(float *dcoef, float *d_scale_bias, const void *dy, int64_t 
 // whatever is fused into it, and a kernel that forms dW tile by tile per block of tokens repeats the k hashes per element for
 // every block.  With room for dW (fp32, [out_f x in_f]) in the caller's workspace it is formed once, by this product, and
 // contracted once by the kernels of rdb_materialize_bwd.  Scratch behind dW: one more [out_f x in_f] matrix per token range.
-static FgPlan dw_plan(const rdb_linear_desc *d, int num_cus) { return fg_plan(d->out_f, d->in_f, d->tokens, num_cus, 256, 64); }
+static int dw_room(const rdb_linear_desc *d, int num_cus) { return fg_room(d->out_f, d->in_f, d->tokens, num_cus, 256, 64).ranges; }
 int64_t linear_dw_f32_workspace(const rdb_linear_desc *d, int num_cus)
 {
     if (d->out_f * d->in_f >= (1ll << 29) || d->tokens <= 0) return 0;
-    const int r = dw_plan(d, num_cus).ranges;
+    const int r = dw_room(d, num_cus);
     return up256(d->out_f * d->in_f * 4) * (1 + (r > 1 ? r : 0));
 }
 int linear_dw_f32(float *dW, const void *dy, int64_t lddy, const void *x, int64_t ldx, const rdb_linear_desc *d, int num_cus, hipStream_t s)
 {
     if (d->tokens * lddy >= (1ll << 29) || d->tokens * ldx >= (1ll << 29) || d->out_f * d->in_f >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     FgProduct q = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, (const float *)x, ldx, (d->tokens - 1) * ldx + d->in_f, dW, d->in_f, nullptr,
-                   d->out_f, d->in_f, d->tokens, 128, 0, 0, d->seed};
+                   d->out_f, d->in_f, d->tokens, 0, 0, 0, 0, d->seed};
     q.a_es = q.b_es = fg_es(d->act_dtype);
     const int64_t stride = up256(d->out_f * d->in_f * 4) / 4;
-    return fg_launch_ranges<FG_MCONT, FG_MCONT>(q, dw_plan(d, num_cus), dW + stride, stride, num_cus, s, "f32_gemm_kernel (dW = dy^T . x)");
+    return fg_launch_ranges<FG_MCONT, FG_MCONT>(q, dw_room(d, num_cus), dW + stride, stride, num_cus, s, "f32_gemm_kernel (dW = dy^T . x)");
 }
 
 // ----------------------------------------------------------------------------------------------- projected form in fp32
@@ -836,14 +960,14 @@ static float *fg_state_z(const void *state) { return reinterpret_cast<float *>(s
 int64_t linear_f32_bwd_projected_workspace(const rdb_linear_desc *d, int num_cus)
 {
     if (!fg_state_ok(d)) return 0;
-    const int r = dc_plan(d, num_cus).ranges;
+    const int r = dc_room(d, num_cus);
     return linear_f32_workspace(RDB_OP_LINEAR_BWD_DX, d, num_cus) + (r > 1 ? (int64_t)r * up256(d->out_f * d->k * 4) : 0);
 }
 
 static int fg_fwd_from_z(void *y, int64_t ldy, const float *z, const void *coef, const void *bias, const rdb_linear_desc *d, int num_cus, hipStream_t s)
 {
     FgProduct q = {z, d->k, d->tokens * d->k, (const float *)coef, d->k, d->out_f * d->k, (float *)y, ldy, (const float *)bias,
-                   d->tokens, d->out_f, d->k, fg_plan(d->tokens, d->out_f, d->k, num_cus, d->k, 1).bm, 0, 0, d->seed};
+                   d->tokens, d->out_f, d->k, 0, 0, 0, 0, d->seed};
     return fg_launch<FG_KCONT, FG_KCONT>(q, num_cus, s, "f32_gemm_kernel (y = z . C^T)");
 }
 
@@ -886,8 +1010,8 @@ int linear_bwd_projected_f32(void *dx, int64_t lddx, float *dcoef, const void *d
     }
     float *part = reinterpret_cast<float *>(static_cast<char *>(workspace) + linear_f32_workspace(RDB_OP_LINEAR_BWD_DX, d, num_cus));
     FgProduct q = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, fg_state_z(state), d->k, d->tokens * d->k, dcoef, d->k, nullptr,
-                   d->out_f, d->k, d->tokens, 128, 0, 0, d->seed};
-    return fg_launch_ranges<FG_MCONT, FG_MCONT>(q, dc_plan(d, num_cus), part, up256(d->out_f * d->k * 4) / 4, num_cus, s,
+                   d->out_f, d->k, d->tokens, 0, 0, 0, 0, d->seed};
+    return fg_launch_ranges<FG_MCONT, FG_MCONT>(q, dc_room(d, num_cus), part, up256(d->out_f * d->k * 4) / 4, num_cus, s,
                                                 "f32_gemm_kernel (dC = dy^T . z)");
 }
 
@@ -912,26 +1036,26 @@ int materialize_mat_f32(float *out, const void *coef, int coef_dtype, int64_t co
     if (!transposed) {
         // W[o, i] = sum_m C[o, m] noise(i, m): rows = o from C, columns = i hashed; the random bias at index o * row_len + i
         FgProduct q = {C, k, coef_rows * k, nullptr, 0, 0, out, row_len, nullptr, coef_rows, row_len, k,
-                       fg_plan(coef_rows, row_len, k, num_cus, k, 1).bm, 0, 0, seed, (uint32_t)row_len, 1u, (const float *)scale_bias, nullptr, 0, nullptr};
+                       0, 0, 0, 0, seed, (uint32_t)row_len, 1u, (const float *)scale_bias, nullptr, 0, nullptr};
         q.a_es = fg_es(coef_dtype);
         q.scale_bf16 = coef_dtype == RDB_BF16;
             return fg_launch<FG_KCONT, FG_NOISE_I>(q, num_cus, s, "f32_gemm_kernel (W = C . N)");
     }
     // W^T[i, o]: rows = i hashed, columns = o from C; the random bias at index o * row_len + i
     FgProduct q = {nullptr, 0, 0, C, k, coef_rows * k, out, coef_rows, nullptr, row_len, coef_rows, k,
-                   fg_plan(row_len, coef_rows, k, num_cus, k, 1).bm, 0, 0, seed, 1u, (uint32_t)row_len, (const float *)scale_bias, nullptr, 0, nullptr};
+                   0, 0, 0, 0, seed, 1u, (uint32_t)row_len, (const float *)scale_bias, nullptr, 0, nullptr};
     q.b_es = fg_es(coef_dtype);
     q.scale_bf16 = coef_dtype == RDB_BF16;
     return fg_launch<FG_NOISE_I, FG_KCONT>(q, num_cus, s, "f32_gemm_kernel (W^T = N^T . C^T)");
 }
 
-static FgPlan mat_bwd_plan(int64_t coef_rows, int64_t k, int64_t row_len, int num_cus) { return fg_plan(coef_rows, k, row_len, num_cus, 256, 64); }
+static int mat_bwd_room(int64_t coef_rows, int64_t k, int64_t row_len, int num_cus) { return fg_room(coef_rows, k, row_len, num_cus, 256, 64).ranges; }
 
 // scratch of the adjoint: one [coef_rows x k] matrix per range of the row (none with a single range)
 int64_t coef_grad_mat_f32_workspace(int64_t coef_rows, int64_t k, int64_t row_len, int num_cus)
 {
     if (!fg_mat_ok(coef_rows, k, row_len, FG_COEF_GRAD_MIN_MACS)) return 0;
-    const int r = mat_bwd_plan(coef_rows, k, row_len, num_cus).ranges;
+    const int r = mat_bwd_room(coef_rows, k, row_len, num_cus);
     return r > 1 ? (int64_t)r * up256(coef_rows * k * 4) : 0;
 }
 
@@ -942,9 +1066,9 @@ int coef_grad_mat_f32(float *dcoef, const void *dW, int dw_dtype, int64_t coef_r
     if (!fg_mat_ok(coef_rows, k, row_len, FG_COEF_GRAD_MIN_MACS)) return RDB_E_UNSUPPORTED;
     const int64_t need = coef_grad_mat_f32_workspace(coef_rows, k, row_len, num_cus);
     if (need > 0 && (!workspace || !fg_aligned16(workspace) || workspace_bytes < need)) return RDB_E_UNSUPPORTED;
-    FgProduct q = {(const float *)dW, row_len, coef_rows * row_len, nullptr, 0, 0, dcoef, k, nullptr, coef_rows, k, row_len, 128, 0, 0, seed};
+    FgProduct q = {(const float *)dW, row_len, coef_rows * row_len, nullptr, 0, 0, dcoef, k, nullptr, coef_rows, k, row_len, 0, 0, 0, 0, seed};
     q.a_es = fg_es(dw_dtype);
-    return fg_launch_ranges<FG_KCONT, FG_NOISE_M>(q, mat_bwd_plan(coef_rows, k, row_len, num_cus), (float *)workspace, up256(coef_rows * k * 4) / 4, num_cus,
+    return fg_launch_ranges<FG_KCONT, FG_NOISE_M>(q, mat_bwd_room(coef_rows, k, row_len, num_cus), (float *)workspace, up256(coef_rows * k * 4) / 4, num_cus,
                                                   s, "f32_gemm_kernel (dcoef = dW . N^T)");
 }
 

@@ -95,6 +95,26 @@ int rdb_scale_bias_bwd(float *ds, const void *dW, int dw_dtype, int64_t Nw, uint
                        void *workspace, int64_t workspace_bytes, void *stream);
 int64_t rdb_scale_bias_bwd_workspace_bytes(int64_t Nw);
 
+/* Gradient of a pseudorandom bias added to every row of a matrix, b[o] = sum_m noise(PRIME*o + m) * coef[m] + s * noise1d(o)
+ * (R.py:979-990 behind the column sums of addmm's backward):  with g[o] = sum_t dy[t, o] in fp32,
+ *   dcoef[m] = sum_o g[o] * noise(PRIME*o + m)   (fp32 [k], overwritten; NULL: not wanted)
+ *   ds[0]    = sum_o g[o] * noise1d(o)           (fp32, overwritten; NULL: not wanted)
+ * dy [rows x n] of `dtype`, unit inner stride.  Sums in a fixed order. */
+int rdb_bias_bwd(float *dcoef, float *ds, const void *dy, int dtype, int64_t ldy, int64_t rows, int64_t n, int64_t k,
+                 uint32_t seed, void *workspace, int64_t workspace_bytes, void *stream);
+int64_t rdb_bias_bwd_workspace_bytes(int64_t rows, int64_t n);
+
+/* ------------------------------------------------------------------------------------------ dense product
+ * The dense products around a materialised weight (aten.mm of R.py:942-946 and its backward), fp32:
+ *   out[M x N] = A . B^T (+ bias[N]),  A [M x K], B [N x K] row-major; a_across / b_across: stored transposed, [K x M] / [K x N].
+ * out is contiguous.  (0, 0), (0, 1) and (1, 1) of the across flags.  On the bf16 matrix cores at fp32 accuracy (three-way
+ * split of both sides, see rdb_set_f32_split); an infinite input becomes NaN.  The workspace holds partial sums over ranges of
+ * K, added in a fixed order; with less of it (or a bias) fewer ranges run.  RDB_E_UNSUPPORTED: empty, or 2^29 elements or more. */
+int rdb_product_f32(float *out, const float *a, int64_t lda, int a_across, const float *b, int64_t ldb, int b_across,
+                    const float *bias, int64_t M, int64_t N, int64_t K, void *workspace, int64_t workspace_bytes,
+                    void *stream);
+int64_t rdb_product_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
+
 /* ------------------------------------------------------------------------------------------ embedding
  * Replaces: op rten::embed_fwd + embed_fwd_kernel (R.py:998-1057, 1121-1126).
  * out[j*rowsize + r] = sum_m noise(PRIME*(idx[j]*rowsize + r) + m) * coef[m];  out fp32 [n_idx x rowsize],

@@ -164,7 +164,9 @@ class SillyLinear(SillyModuleMixin, nn.Module):
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:
         if not self.fused:
-            return F.linear(input, self.weight, self.bias)
+            w, b = self.weight, self.bias
+            y = ops.vector_linear(input, w, b) if isinstance(w, RandumbTensor) and not (w.FUSED_MM and w.FUSED_MM_VECTOR) else None
+            return F.linear(input, w, b) if y is None else y
         in_f, out_f = self.in_features, self.out_features
         w = self._buffers["weight"]   # past nn.Module's attribute search: a few-token layer's kernels take less than a forward's host time
         flat = input.dim() == 2
@@ -246,7 +248,7 @@ class SillyEmbedding(SillyModuleMixin, nn.Module):
         init_kaiming_uniform(self.weight, None, seed=self.seed[0])
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:
-        return ops.embed_fwd(input, self.weight_coef, self.embedding_dim, self.weight.seed)
+        return ops.embed_rows(input, self.weight_coef, self.embedding_dim, self.weight.seed)
 
     def extra_repr(self) -> str:
         return f"{self.num_embeddings}, {self.embedding_dim}, int_dim={self.int_dim}, seeds={self.seed}"

@@ -29,6 +29,10 @@ EXPORTS = [
     "rdb_materialize_bwd_workspace_bytes",
     "rdb_scale_bias_bwd",
     "rdb_scale_bias_bwd_workspace_bytes",
+    "rdb_bias_bwd",
+    "rdb_bias_bwd_workspace_bytes",
+    "rdb_product_f32",
+    "rdb_product_f32_workspace_bytes",
     "rdb_embed_fwd",
     "rdb_embed_bwd",
     "rdb_embed_bwd_workspace_bytes",
@@ -145,6 +149,14 @@ def load() -> ctypes.CDLL:
     L.rdb_scale_bias_bwd.argtypes = [vp, vp, ci, i64, u32, vp, i64, vp]
     L.rdb_scale_bias_bwd_workspace_bytes.argtypes = [i64]
     L.rdb_scale_bias_bwd_workspace_bytes.restype = i64
+    L.rdb_bias_bwd.argtypes = [vp, vp, vp, ci, i64, i64, i64, i64, u32, vp, i64, vp]
+    L.rdb_bias_bwd.restype = ci
+    L.rdb_bias_bwd_workspace_bytes.argtypes = [i64, i64]
+    L.rdb_bias_bwd_workspace_bytes.restype = i64
+    L.rdb_product_f32.argtypes = [vp, vp, i64, ci, vp, i64, ci, vp, i64, i64, i64, vp, i64, vp]
+    L.rdb_product_f32.restype = ci
+    L.rdb_product_f32_workspace_bytes.argtypes = [i64, i64, i64]
+    L.rdb_product_f32_workspace_bytes.restype = i64
     L.rdb_embed_fwd.argtypes = [vp, vp, i64, vp, ci, i64, i64, u32, vp]
     L.rdb_embed_bwd.argtypes = [vp, vp, i64, vp, ci, i64, i64, u32, vp, i64, vp]
     L.rdb_embed_bwd_workspace_bytes.argtypes = [i64, i64, i64]

@@ -18,511 +18,11 @@
 // the gradient of s is <dy, x . R^T>, summed tile by tile in the epilogue of that product and block by block afterwards.
 // Replaces materialize() + dense product (src/rten_cpp/RandumbTensor.py:942-946) and MmBackward's dW followed by
 // materialize_bwd (RandumbTensor.py:979-990, 304-359) for fp32 layers beyond the few-token regime of rdb_smallk.hip.
-#include "rdb_gemm.hpp"
-#include <algorithm>
-#include <type_traits>
+#include "rdb_f32.hpp"
 
 namespace rdb {
 
-constexpr int FG_BN = 128;        // B rows (output columns) per block
-constexpr int FG_BK = 16;         // contraction values per stage
-constexpr int FG_THREADS = 256;   // threads of a group: four waves, 2 x 2
-constexpr uint32_t FG_OOB = 0x80000000u;   // a byte offset past the end of any matrix these kernels take (below 2^31 bytes)
-
-// Where an operand's tile [rows x FG_BK] comes from.  In LDS every tile is [FG_BK][rows + 4]: an MFMA operand is 32
-// consecutive floats of each of two contraction values.
-enum FgSource {
-    FG_KCONT = 0,    // src[row * ld + kk]: a row-major matrix whose rows are the tile's rows
-    FG_MCONT = 1,    // src[kk * ld + row]: a row-major matrix whose rows are contraction values
-    FG_NOISE_M = 2,  // 2-D noise (feature kk, coefficient row): the rows are coefficients, the contraction runs over features
-    FG_NOISE_I = 3,  // 2-D noise (feature row, coefficient kk): the rows are features, the contraction runs over coefficients
-    FG_NOISE_1D = 4  // 1-D noise at index row * sR + kk * sK: the random-bias matrix R, read along or across its rows
-};
-// What a block does with its accumulators.
-enum FgEpilogue {
-    FG_STORE = 0,       // out = acc
-    FG_STORE_BIAS = 1,  // out = acc + bias[column]
-    FG_ADD_SCALED = 2,  // out += scale[0] * acc
-    FG_DOT = 3,         // dot_part[block] = sum over the tile of acc * dotm (nothing is stored to out)
-    FG_STORE_RBIAS = 4  // out = acc + scale[0] * noise1d(row * nsR + column * nsK): materialising W = C . N + s . R
-};
-
-struct FgParams {
-    const float *a;   // A operand's matrix (FG_KCONT / FG_MCONT)
-    int64_t lda;
-    const float *b;   // B operand's matrix; not used by the noise sources
-    int64_t ldb;
-    float *out;       // [M x N], leading dimension ldo; split s of the contraction writes out + s * split_stride
-    int64_t ldo, split_stride;
-    const float *bias;   // [N] or NULL
-    int M, N, K;
-    int kchunk;          // contraction values per split (a multiple of FG_BK); K when there is one split
-    int64_t a_bytes, b_bytes;   // extent of the matrices, for the bounds check of the loads (< 2^31)
-    uint32_t seed;
-    int a_es, b_es;             // bytes per element of the A and B matrices: 4, or 2 (bf16; only the value-by-value kernels)
-    int out_bf16;               // out, bias and dotm are bf16 (the activations' dtype)
-    int scale_bf16;             // scale is bf16 (the coefficients' dtype)
-    uint32_t nsR, nsK;          // FG_NOISE_1D: index steps per row and per contraction value
-    const float *scale;         // FG_ADD_SCALED: one device value
-    const float *dotm;          // FG_DOT: [M x N] matrix, leading dimension lddot
-    int64_t lddot;
-    float *dot_part;            // FG_DOT: one value per block, in block order (x fastest, then y)
-};
-
-// fp32 products on the bf16 matrix cores.  v = h + m + l exactly, each part a bf16 (the top 8 bits of what is left: truncation,
-// so every difference is exact); a product a . b is then the sum of the nine products of the parts, each exact in the matrix
-// core's fp32 accumulation, and the six largest of them, ah bh + ah bm + am bh + ah bl + al bh + am bm, leave out less than
-// 2^-23 |a b|: an fp32 product's own rounding.  Six bf16 matrix instructions of 32 x 32 x 16 do the work of eight fp32 ones of
-// 32 x 32 x 2 in 3/8 of the time.  (An infinite input becomes NaN: inf - inf.)  The parts come back as fp32 bit patterns with
-// the low half zero.
-__device__ __forceinline__ void fg_split3(float v, uint32_t &h, uint32_t &m, uint32_t &l)
-{
-    h = __float_as_uint(v) & 0xffff0000u;
-    const float r1 = v - __uint_as_float(h);
-    m = __float_as_uint(r1) & 0xffff0000u;
-    const float r2 = r1 - __uint_as_float(m);
-    l = __float_as_uint(r2) & 0xffff0000u;
-}
-
-// One operand's way from its source into LDS: load(stage) requests / hashes the stage's values into registers, store() puts
-// them into a tile.  Rows past `rows` and contraction values past `kend` are zeros.
-// VEC: the matrix is read in pieces of four values (16 bytes of fp32, 8 bytes of bf16; 16-byte aligned base, leading dimension a
-// multiple of 4, and the extent that runs along a piece a multiple of 4, so that a piece lies inside or outside as a whole);
-// otherwise four values at a time at any address where all four exist, value by value at the edges.
-// SPLIT: the tile goes to LDS as three bf16 planes (see fg_split3): planes of [2 halves of the stage's 16 contraction values]
-// [rows][8] for the sources read along the contraction (a lane's MFMA operand is 16 consecutive bytes), of [16][rows + 32] for
-// FG_MCONT (read back with the LDS transpose read).  The noise sources then give a thread consecutive contraction values.
-template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
-    static constexpr int LD = ROWS + 4, TILE = FG_BK * LD, NV = ROWS * FG_BK / FG_THREADS / 4;   // float4 per thread and stage
-    static_assert(NV >= 1, "a stage is at least one float4 per thread");
-    static constexpr int LDM = ROWS + 32;                                            // FG_MCONT plane: elements per contraction value
-    static constexpr int PLANE = SRC == FG_MCONT ? FG_BK * LDM : 2 * ROWS * 8;       // bf16 elements of one plane
-    static constexpr int TILE_BYTES = SPLIT ? 3 * PLANE * 2 : TILE * 4;
-    static constexpr int KPT = NV * 4;                                               // SPLIT, noise: consecutive contraction values per thread
-    __amdgpu_buffer_rsrc_t rs;
-    uint32_t off[NV];   // byte offset of the thread's pieces at stage 0
-    bool ok[NV];        // ... and whether the piece's (first) row exists
-    uint32_t step;      // bytes per stage
-    uint32_t first;     // noise: first-round value of the thread's first element at stage 0
-    int kk0, kend, k_begin, row_ok;
-    int rows_left[NV];  // FG_MCONT without VEC: how many of the piece's four rows exist
-    f32x4 r[NV];
-
-    uint32_t inc;       // noise: first-round step per contraction value
-    const char *base;   // the matrix, for load4u
-    int es;             // bytes per element of the matrix (2: bf16)
-    __device__ __forceinline__ float load1(uint32_t o, bool in, int j) const
-    {
-        if (es == 2) {
-            const unsigned short h = __builtin_amdgcn_raw_buffer_load_b16(rs, in ? (int)(o + 2 * j) : (int)FG_OOB, 0, 0);
-            return bf16_to_f32(h);
-        }
-        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, in ? (int)(o + 4 * j) : (int)FG_OOB, 0, 0));
-    }
-    // VEC: four consecutive elements at byte offset o (fp32: 16 bytes; bf16: 8 bytes, widened), zeros when outside
-    __device__ __forceinline__ f32x4 load4(uint32_t o, bool in) const
-    {
-        if (es == 2) {
-            const f32x2 h = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, in ? (int)o : (int)FG_OOB, 0, 0));
-            const uint32_t lo = __float_as_uint(h[0]), hi = __float_as_uint(h[1]);
-            return f32x4{__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u), __uint_as_float(hi << 16), __uint_as_float(hi & 0xffff0000u)};
-        }
-        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, in ? (int)o : (int)FG_OOB, 0, 0));
-    }
-    // not VEC: four consecutive elements that all exist, at any element's address (the hardware takes loads of 8 and 16 bytes at
-    // any address; 4097 tokens x 1001 features in bf16, k = 100: z = x . N^T 20.8 us with a load per value, 14.4 us with these)
-    __device__ __forceinline__ f32x4 load4u(uint32_t o) const
-    {
-        if (es == 2) {
-            typedef uint32_t pair_any __attribute__((ext_vector_type(2), aligned(2)));
-            const pair_any h = *reinterpret_cast<const pair_any *>(base + o);
-            return f32x4{__uint_as_float(h[0] << 16), __uint_as_float(h[0] & 0xffff0000u), __uint_as_float(h[1] << 16), __uint_as_float(h[1] & 0xffff0000u)};
-        }
-        typedef float quad_any __attribute__((ext_vector_type(4), aligned(4)));
-        const quad_any v = *reinterpret_cast<const quad_any *>(base + o);
-        return f32x4{v[0], v[1], v[2], v[3]};
-    }
-    __device__ __forceinline__ void init(const float *src, int64_t ld, int64_t bytes, int row0, int rows, int k_begin_, int kend_, uint32_t seed,
-                                         uint32_t sR, uint32_t sK, int es_)
-    {
-        const int t = threadIdx.x & (FG_THREADS - 1);
-        k_begin = k_begin_;
-        kend = kend_;
-        es = es_;
-        base = reinterpret_cast<const char *>(src);
-        if (SRC == FG_KCONT) {
-            rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(src), 0, (int)bytes, 0x00020000);
-            step = (uint32_t)(FG_BK * es);
-#pragma unroll
-            for (int h = 0; h < NV; ++h) {
-                const int idx = h * FG_THREADS + t, row = idx >> 2, kq = idx & 3;
-                ok[h] = row0 + row < rows;
-                off[h] = ok[h] ? (uint32_t)(((int64_t)(row0 + row) * ld + k_begin + kq * 4) * es) : 0u;
-            }
-            kk0 = (t & 3) * 4;
-        } else if (SRC == FG_MCONT) {
-            rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(src), 0, (int)bytes, 0x00020000);
-            step = (uint32_t)(FG_BK * ld * es);
-#pragma unroll
-            for (int h = 0; h < NV; ++h) {
-                const int idx = h * FG_THREADS + t, kk = idx / (ROWS / 4), r4 = (idx % (ROWS / 4)) * 4;
-                ok[h] = row0 + r4 < rows;
-                off[h] = ok[h] ? (uint32_t)(((int64_t)(k_begin + kk) * ld + row0 + r4) * es) : 0u;
-                rows_left[h] = rows - (row0 + r4);
-            }
-            kk0 = t / (ROWS / 4);
-        } else {
-            const int row = t % ROWS;
-            kk0 = SPLIT ? (t / ROWS) * KPT : t / ROWS;
-            row_ok = row0 + row < rows;
-            if (SRC == FG_NOISE_1D) {
-                first = ((uint32_t)(row0 + row) * sR + (uint32_t)(k_begin + kk0) * sK) * SQ5_N1 + seed;
-                inc = sK * SQ5_N1;
-            } else {
-                first = SRC == FG_NOISE_M ? sq5_first((uint32_t)(k_begin + kk0), (uint32_t)(row0 + row), seed)
-                                          : sq5_first((uint32_t)(row0 + row), (uint32_t)(k_begin + kk0), seed);
-                inc = SRC == FG_NOISE_M ? PN1 : SQ5_N1;
-            }
-        }
-    }
-    __device__ __forceinline__ void load(int stage)
-    {
-        if (SRC == FG_KCONT) {
-            // a thread's four values are consecutive contraction values
-            const int kk = k_begin + stage * FG_BK + kk0;
-#pragma unroll
-            for (int h = 0; h < NV; ++h) {
-                const uint32_t o = off[h] + (uint32_t)stage * step;
-                if (VEC) {   // all inside or all outside
-                    r[h] = load4(o, ok[h] && kk < kend);
-                } else if (ok[h] && kk + 4 <= kend) {
-                    r[h] = load4u(o);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) r[h][j] = load1(o, ok[h] && kk + j < kend, j);
-                }
-            }
-        } else if (SRC == FG_MCONT) {
-#pragma unroll
-            for (int h = 0; h < NV; ++h) {
-                const bool in = ok[h] && k_begin + stage * FG_BK + kk0 + h * (FG_THREADS / (ROWS / 4)) < kend;
-                const uint32_t o = off[h] + (uint32_t)stage * step;
-                if (VEC) {
-                    r[h] = load4(o, in);
-                } else if (in && rows_left[h] >= 4) {
-                    r[h] = load4u(o);
-                } else {   // a thread's four values are consecutive rows: rows_left of them exist
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) r[h][j] = load1(o, in && j < rows_left[h], j);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < NV * 4; ++j) hash_piece(stage, j);
-        }
-    }
-    // Noise sources: element j of the thread's NV * 4 values of a stage (contraction value kk0 + j * (FG_THREADS / ROWS), one add
-    // apart in the first round).  The main loop calls this between the matrix instructions of the stage before.
-    static constexpr bool HASHED = SRC == FG_NOISE_M || SRC == FG_NOISE_I || SRC == FG_NOISE_1D;
-    __device__ __forceinline__ void hash_piece(int stage, int j)
-    {
-        constexpr int KSTEP = SPLIT ? 1 : FG_THREADS / ROWS;
-        const uint32_t f = first + (uint32_t)(stage * FG_BK + j * KSTEP) * inc;
-        const bool in = row_ok && k_begin + stage * FG_BK + kk0 + j * KSTEP < kend;
-        r[j >> 2][j & 3] = in ? sq5_unit(sq5_tail(f)) : 0.0f;
-    }
-    __device__ __forceinline__ void store(float *__restrict__ tile) const
-    {
-        const int t = threadIdx.x & (FG_THREADS - 1);
-        if (SRC == FG_KCONT) {
-#pragma unroll
-            for (int h = 0; h < NV; ++h) {
-                const int idx = h * FG_THREADS + t, row = idx >> 2, kq = idx & 3;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) tile[(kq * 4 + j) * LD + row] = r[h][j];
-            }
-        } else if (SRC == FG_MCONT) {
-#pragma unroll
-            for (int h = 0; h < NV; ++h) {
-                const int idx = h * FG_THREADS + t, kk = idx / (ROWS / 4), r4 = (idx % (ROWS / 4)) * 4;
-                *reinterpret_cast<f32x4 *>(tile + kk * LD + r4) = r[h];
-            }
-        } else {
-            constexpr int KSTEP = FG_THREADS / ROWS;
-            const int row = t % ROWS;
-#pragma unroll
-            for (int j = 0; j < NV * 4; ++j) tile[(kk0 + j * KSTEP) * LD + row] = r[j >> 2][j & 3];
-        }
-    }
-    // SPLIT: four of the thread's values into the planes, 8 bytes each, at element offset `at` of a plane.  Values that come from a
-    // bf16 matrix are their own first part and the other two are zero: only the first plane is written (and read, see the kernel).
-    __device__ __forceinline__ bool one_plane() const { return !HASHED && es == 2; }
-    template <bool ONE> __device__ __forceinline__ void put4(bf16_t *__restrict__ tile, int at, const f32x4 &v) const
-    {
-        if (ONE) {
-            *reinterpret_cast<uint2 *>(tile + at) = make_uint2((__float_as_uint(v[1]) & 0xffff0000u) | (__float_as_uint(v[0]) >> 16),
-                                                               (__float_as_uint(v[3]) & 0xffff0000u) | (__float_as_uint(v[2]) >> 16));
-            return;
-        }
-        uint32_t h[4], m[4], l[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) fg_split3(v[j], h[j], m[j], l[j]);
-        *reinterpret_cast<uint2 *>(tile + at) = make_uint2(h[1] | (h[0] >> 16), h[3] | (h[2] >> 16));
-        *reinterpret_cast<uint2 *>(tile + PLANE + at) = make_uint2(m[1] | (m[0] >> 16), m[3] | (m[2] >> 16));
-        *reinterpret_cast<uint2 *>(tile + 2 * PLANE + at) = make_uint2(l[1] | (l[0] >> 16), l[3] | (l[2] >> 16));
-    }
-    template <bool ONE> __device__ __forceinline__ void store_split(bf16_t *__restrict__ tile) const
-    {
-        const int t = threadIdx.x & (FG_THREADS - 1);
-        if (SRC == FG_KCONT) {
-#pragma unroll
-            for (int h = 0; h < NV; ++h) {   // contraction values 4 kq .. 4 kq + 3 of a row
-                const int idx = h * FG_THREADS + t, row = idx >> 2, kq = idx & 3;
-                put4<ONE>(tile, ((kq >> 1) * ROWS + row) * 8 + (kq & 1) * 4, r[h]);
-            }
-        } else if (SRC == FG_MCONT) {
-#pragma unroll
-            for (int h = 0; h < NV; ++h) {   // four consecutive rows at one contraction value
-                const int idx = h * FG_THREADS + t, kk = idx / (ROWS / 4), r4 = (idx % (ROWS / 4)) * 4;
-                put4<ONE>(tile, kk * LDM + r4, r[h]);
-            }
-        } else {
-            const int row = t % ROWS;
-#pragma unroll
-            for (int h = 0; h < NV; ++h) {   // contraction values kk0 + 4 h .. + 3 of a row
-                const int kk = kk0 + 4 * h;
-                put4<ONE>(tile, ((kk >> 3) * ROWS + row) * 8 + (kk & 7), r[h]);
-            }
-        }
-    }
-    // SPLIT: the MFMA operand of the 32 rows from rb of one plane: lane (r, g) gets contraction values 8 g .. 8 g + 7 of row rb + r
-    __device__ static __forceinline__ bf16x8 frag(const bf16_t *__restrict__ plane, int rb, int lane)
-    {
-        const int r = lane & 31, g = lane >> 5;
-        if (SRC != FG_MCONT) return *reinterpret_cast<const bf16x8 *>(plane + (g * ROWS + rb + r) * 8);
-        // 16-lane group q covers rows rb + 16 q .. + 15; source lane s of the group addresses contraction value 8 g + s / 4,
-        // rows 4 (s % 4) .. + 3; result lane c receives the rows' column c for four contraction values
-        Frag8 f;
-        const int sl = lane & 15, q = (lane >> 4) & 1;
-        const bf16_t *src = plane + (g * 8 + (sl >> 2)) * LDM + rb + q * 16 + (sl & 3) * 4;
-        f.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)(src));
-        f.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)(src + 4 * LDM));
-        return f.v;
-    }
-};
-
-// out[M x N] (+)= A . B^T over one split of the contraction.  Block: BM x 128 of the output, G groups of four waves as 2 x 2, a
-// wave owns (BM / 2) x 64 in BM / 64 x 2 accumulator tiles.  Two LDS buffers, one barrier per stage: while a stage is multiplied
-// the next one is on its way from memory (or being hashed) in registers.
-// G groups cut the block's contraction into G runs of stages, each with its own LDS buffers, and add their accumulators up
-// through LDS in group order at the end.  One group is one wave to a SIMD, and its stages are a serial chain of about 1 us (load,
-// split, barrier, LDS read, products, hash): a product with fewer blocks than compute units is bound by that chain, and G of
-// them run side by side.  2048 tokens x 768 -> 3072, k = 256, fp32: z = x . N^T 14.6 us (64 rows, 6 ranges) -> 10.3 (G = 4, 4
-// ranges), dx = t . N 19.5 -> 11.7 (G = 4), t = dy . C 27.4 us in 16 ranges -> 23.4 in 8 (G = 2: half the partial sums).  With
-// blocks enough the chip's power is the bound (1.75 GHz under y = z . C^T, 3 groups a unit), and how the groups are arranged
-// matters little.
-// Results leave with streaming stores: they would be written back from L2 at the end of the kernel otherwise, after the last
-// block (y of that layer, 25 MB: 26.4 -> 24.8 us).
-template <int BM, int G, int ASRC, int BSRC, int EPI, bool VEC, bool SPLIT = false, bool ANY16 = false>
-__global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kernel(FgParams p)
-{
-    typedef FgOperand<BM, ASRC, VEC, SPLIT> PA;
-    typedef FgOperand<FG_BN, BSRC, VEC, SPLIT> PB;
-    constexpr int MI = BM / 64, NI = 2, STAGE = (PA::TILE_BYTES + PB::TILE_BYTES) / 4;   // floats
-    static_assert(G == 1 || SPLIT, "groups: the bf16 matrix instructions only");
-    constexpr int UNITS = MI * NI * 2;   // a wave's accumulators in units of 8 registers: what the groups share out at the end
-    constexpr int EXCHANGE = (G - 1) * UNITS * 4 * 512;
-    __shared__ __align__(16) float lds_all[2 * STAGE * G > EXCHANGE ? 2 * STAGE * G : EXCHANGE];
-    const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / FG_THREADS);
-    float *lds = lds_all + group * 2 * STAGE;
-    const int t = threadIdx.x & (FG_THREADS - 1), wave = t >> 6, lane = t & 63, r = lane & 31, g = lane >> 5, wm = wave >> 1, wn = wave & 1;
-    const int m0 = blockIdx.x * BM, n0 = blockIdx.y * FG_BN;   // the long extent (tokens, as a rule) on the grid's x
-    const int k_first = blockIdx.z * p.kchunk, k_last = min(p.K, k_first + p.kchunk);
-    const int nstage = ((k_last - k_first + FG_BK - 1) / FG_BK + G - 1) / G;   // of every group: the last one's may be empty
-    const int k_begin = k_first + group * nstage * FG_BK, kend = min(k_last, k_begin + nstage * FG_BK);
-    PA pa;
-    PB pb;
-    pa.init(p.a, p.lda, p.a_bytes, m0, p.M, k_begin, kend, p.seed, p.nsR, p.nsK, p.a_es);
-    pb.init(p.b, p.ldb, p.b_bytes, n0, p.N, k_begin, kend, p.seed, p.nsR, p.nsK, p.b_es);
-    f32x16 acc[MI][NI];
-#pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < NI; ++ni)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[mi][ni][e] = 0.0f;
-    pa.load(0);
-    pb.load(0);
-    // The stage loop, once per number of planes of the two sides (known per launch, not per kernel: a side that comes from a
-    // bf16 matrix has one plane), so that each copy is straight-line code between its barriers.
-    auto stages = [&](auto a_one, auto b_one) __attribute__((always_inline)) {
-        constexpr int AP = decltype(a_one)::value ? 1 : 3, BP = decltype(b_one)::value ? 1 : 3;
-        for (int s = 0; s < nstage; ++s) {
-            float *As = lds + (s & 1) * STAGE, *Bs = As + PA::TILE_BYTES / 4;
-            if (SPLIT) {
-                pa.template store_split<AP == 1>(reinterpret_cast<bf16_t *>(As));
-                pb.template store_split<BP == 1>(reinterpret_cast<bf16_t *>(Bs));
-            } else {
-                pa.store(As);
-                pb.store(Bs);
-            }
-            __syncthreads();   // also: every wave is done reading the other buffer (the stage before this one)
-            const bool more = s + 1 < nstage;
-            if (more) {
-                if (!PA::HASHED) pa.load(s + 1);
-                if (!PB::HASHED) pb.load(s + 1);
-            }
-            if (SPLIT) {
-                // the stage is one k-step of the bf16 matrix instruction: three planes a side, six products a tile pair, the small
-                // ones first (a side that comes from a bf16 matrix has one plane: three products, or one); the next stage's noise
-                // values are hashed between the tile pairs
-                const bf16_t *ap = reinterpret_cast<const bf16_t *>(As), *bp = reinterpret_cast<const bf16_t *>(Bs);
-                {
-                    bf16x8 fa[MI][AP], fb[NI][BP];
-#pragma unroll
-                    for (int pl = 0; pl < 3; ++pl) {
-#pragma unroll
-                        for (int mi = 0; mi < MI; ++mi)
-                            if (pl < AP) fa[mi][pl] = PA::frag(ap + pl * PA::PLANE, wm * (BM / 2) + mi * 32, lane);
-#pragma unroll
-                        for (int ni = 0; ni < NI; ++ni)
-                            if (pl < BP) fb[ni][pl] = PB::frag(bp + pl * PB::PLANE, wn * 64 + ni * 32, lane);
-                    }
-#pragma unroll
-                    for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-                        for (int ni = 0; ni < NI; ++ni) {
-                            f32x16 c = acc[mi][ni];
-                            if constexpr (AP == 3 && BP == 3) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][1], fb[ni][1], c, 0, 0, 0);
-                            if constexpr (AP == 3) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][2], fb[ni][0], c, 0, 0, 0);
-                            if constexpr (BP == 3) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][0], fb[ni][2], c, 0, 0, 0);
-                            if constexpr (AP == 3) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][1], fb[ni][0], c, 0, 0, 0);
-                            if constexpr (BP == 3) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][0], fb[ni][1], c, 0, 0, 0);
-                            acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][0], fb[ni][0], c, 0, 0, 0);
-                            constexpr int GROUPS = MI * NI;
-                            const int grp = mi * NI + ni;
-                            if (PB::HASHED && more) {
-                                constexpr int PER = (PB::NV * 4 + GROUPS - 1) / GROUPS;
-#pragma unroll
-                                for (int j = grp * PER; j < (grp + 1) * PER && j < PB::NV * 4; ++j) pb.hash_piece(s + 1, j);
-                            }
-                            if (PA::HASHED && more) {
-                                constexpr int PER = (PA::NV * 4 + GROUPS - 1) / GROUPS;
-#pragma unroll
-                                for (int j = grp * PER; j < (grp + 1) * PER && j < PA::NV * 4; ++j) pa.hash_piece(s + 1, j);
-                            }
-                        }
-                }
-                continue;
-            }
-            const float *ap = As + g * PA::LD + wm * (BM / 2) + r, *bp = Bs + g * PB::LD + wn * 64 + r;
-#pragma unroll
-            for (int ks = 0; ks < FG_BK / 2; ++ks) {
-                float fa[MI], fb[NI];
-#pragma unroll
-                for (int mi = 0; mi < MI; ++mi) fa[mi] = ap[ks * 2 * PA::LD + mi * 32];
-#pragma unroll
-                for (int ni = 0; ni < NI; ++ni) fb[ni] = bp[ks * 2 * PB::LD + ni * 32];
-#pragma unroll
-                for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-                    for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[mi], fb[ni], acc[mi][ni], 0, 0, 0);
-                // the next stage's noise values are hashed in the shadow of these matrix instructions, a share per k-step
-                if (PB::HASHED && more) {
-                    constexpr int PER = (PB::NV * 4 + FG_BK / 2 - 1) / (FG_BK / 2);
-#pragma unroll
-                    for (int j = ks * PER; j < (ks + 1) * PER && j < PB::NV * 4; ++j) pb.hash_piece(s + 1, j);
-                }
-                if (PA::HASHED && more) {
-                    constexpr int PER = (PA::NV * 4 + FG_BK / 2 - 1) / (FG_BK / 2);
-#pragma unroll
-                    for (int j = ks * PER; j < (ks + 1) * PER && j < PA::NV * 4; ++j) pa.hash_piece(s + 1, j);
-                }
-            }
-        }
-    };
-    typedef std::integral_constant<bool, true> One;
-    typedef std::integral_constant<bool, false> Three;
-    if (!SPLIT || !ANY16) {   // ANY16: one of the matrices is bf16 (only then is the choice compiled in)
-        stages(Three{}, Three{});
-    } else {
-        const bool a1 = pa.one_plane(), b1 = pb.one_plane();
-        if (PA::HASHED || !a1) {
-            if (PB::HASHED || !b1) stages(Three{}, Three{});
-            else stages(Three{}, One{});
-        } else {
-            if (PB::HASHED || !b1) stages(One{}, Three{});
-            else stages(One{}, One{});
-        }
-    }
-    if constexpr (G > 1) {
-        // unit u (registers 8 (u % 2) .. of tile u / 2) is finished by group u * G / UNITS; the others hand theirs over
-        __syncthreads();   // the stage buffers are free
-        auto slot = [&](int u, int from, int owner) { return lds_all + ((u * (G - 1) + (from < owner ? from : from - 1)) * 4 + wave) * 512 + lane; };
-#pragma unroll
-        for (int u = 0; u < UNITS; ++u) {
-            const int owner = u * G / UNITS;
-            if (group == owner) continue;
-            float *dst = slot(u, group, owner);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) dst[j * 64] = acc[u / 2 / NI][u / 2 % NI][(u & 1) * 8 + j];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < UNITS; ++u) {
-            const int owner = u * G / UNITS;
-            if (group != owner) continue;
-#pragma unroll
-            for (int from = 0; from < G; ++from) {
-                if (from == owner) continue;
-                const float *src = slot(u, from, owner);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) acc[u / 2 / NI][u / 2 % NI][(u & 1) * 8 + j] += src[j * 64];
-            }
-        }
-    }
-    // accumulator j of lane (r, g): row 8 (j / 4) + 4 g + j % 4 of the A side, column r of the B side
-    float *out = p.out + (int64_t)blockIdx.z * p.split_stride;
-    bf16_t *out16 = reinterpret_cast<bf16_t *>(p.out);   // bf16 outputs are never the ranges' partial matrices
-    const bool o16 = p.out_bf16 != 0;
-    const float scale = (EPI != FG_ADD_SCALED && EPI != FG_STORE_RBIAS) ? 0.0f
-                        : p.scale_bf16 ? bf16_to_f32(reinterpret_cast<const bf16_t *>(p.scale)[0]) : p.scale[0];
-    float dot = 0.0f;
-#pragma unroll
-    for (int ni = 0; ni < NI; ++ni) {
-        const int n = n0 + wn * 64 + ni * 32 + r;
-        if (n >= p.N) continue;
-        const float bv = EPI != FG_STORE_BIAS ? 0.0f : o16 ? bf16_to_f32(reinterpret_cast<const bf16_t *>(p.bias)[n]) : p.bias[n];
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                if (G > 1 && group != ((mi * NI + ni) * 2 + j / 8) * G / UNITS) continue;
-                const int m = m0 + wm * (BM / 2) + mi * 32 + 8 * (j >> 2) + 4 * g + (j & 3);
-                if (m >= p.M) continue;
-                const float a = acc[mi][ni][j];
-                if (EPI == FG_DOT) {
-                    const int64_t e = (int64_t)m * p.lddot + n;
-                    dot = fmaf(a, o16 ? bf16_to_f32(reinterpret_cast<const bf16_t *>(p.dotm)[e]) : p.dotm[e], dot);
-                } else {
-                    const int64_t e = (int64_t)m * p.ldo + n;
-                    if (EPI == FG_STORE_RBIAS) out[e] = fmaf(scale, noise1d((uint32_t)m * p.nsR + (uint32_t)n * p.nsK, p.seed), a);
-                    else if (o16) out16[e] = f32_to_bf16(EPI == FG_ADD_SCALED ? fmaf(scale, a, bf16_to_f32(out16[e])) : a + bv);
-                    else if (EPI == FG_ADD_SCALED) out[e] = fmaf(scale, a, out[e]);
-                    else __builtin_nontemporal_store(a + bv, out + e);
-                }
-            }
-    }
-    if (EPI == FG_DOT) {
-        // lanes, then waves, in a fixed order
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) dot += __shfl_xor(dot, o);
-        __syncthreads();   // the stage buffers are free
-        if (lane == 0) lds[wave] = dot;
-        __syncthreads();
-        if (t == 0) p.dot_part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = (lds[0] + lds[1]) + (lds[2] + lds[3]);
-    }
-}
+int num_compute_units();   // rdb_error.hip
 
 // out[0] = part[0] + part[1] + ... : one block, every thread a strided share in index order, then the shares in thread order
 __global__ __launch_bounds__(256) void f32_sum_scalars_kernel(float *__restrict__ out, const float *__restrict__ part, int n)
@@ -559,9 +59,16 @@ __global__ __launch_bounds__(256) void f32_sum_splits_kernel(void *__restrict__ 
     }
 }
 
-// ----------------------------------------------------------------------------------------------- host side
-static bool fg_aligned16(const void *q) { return ((uintptr_t)q & 15) == 0; }
-static int64_t up256(int64_t n) { return (n + 255) / 256 * 256; }
+// 1 (default): the linear layers' products run as six bf16 matrix instructions on three-way splits of their operands
+// (fg_split3); 0: as fp32 matrix instructions.  Process-wide (rdb_set_f32_split).
+static int g_f32_split = 1;
+int f32_split_mode() { return g_f32_split; }
+int set_f32_split_mode(int mode)
+{
+    const int old = g_f32_split;
+    g_f32_split = mode ? 1 : 0;
+    return old;
+}
 
 // The shapes these kernels take: matrix-coef fp32, matrices below 2^31 bytes.  Extents, leading dimensions and pointers that are
 // multiples of 4 elements / 16 bytes get the kernels that read 16 bytes at a time, everything else the value-by-value ones.
@@ -576,77 +83,6 @@ static int fg_es(int dtype) { return dtype == RDB_BF16 ? 2 : 4; }
 // few TFLOP/s, so the factored form on the matrix cores wins also where it is more flops than a product on a stored W.
 static bool fg_wanted(const rdb_linear_desc *) { return true; }
 
-// 1 (default): the linear layers' products run as six bf16 matrix instructions on three-way splits of their operands
-// (fg_split3); 0: as fp32 matrix instructions.  Process-wide (rdb_set_f32_split).
-static int g_f32_split = 1;
-int f32_split_mode() { return g_f32_split; }
-int set_f32_split_mode(int mode)
-{
-    const int old = g_f32_split;
-    g_f32_split = mode ? 1 : 0;
-    return old;
-}
-
-// How a product [M x N] over K runs: tile height, groups per block, contraction ranges.  Each range leaves a partial matrix,
-// added up in range order afterwards, so the result does not depend on which block finishes first.
-struct FgPlan {
-    int bm, ranges, groups;
-};
-// Room for partial matrices: what a workspace holds.  128-row tiles, two blocks per compute unit at a time, unless even in ranges
-// they would leave half of the compute units without a block; 64-row tiles then.  A product with fewer tiles than that is cut
-// into ranges of the contraction, at least min_range values each, at most max_ranges.
-static FgPlan fg_room(int64_t M, int64_t N, int64_t K, int num_cus, int64_t min_range, int max_ranges)
-{
-    const int64_t slots = 2 * (int64_t)num_cus;
-    const int64_t t128 = cdiv(M, 128) * cdiv(N, FG_BN), t64 = cdiv(M, 64) * cdiv(N, FG_BN);
-    int64_t cap = K / min_range;
-    if (cap > max_ranges) cap = max_ranges;
-    if (cap < 1) cap = 1;
-    auto ranges = [&](int64_t tiles) {
-        int64_t r = slots / tiles;
-        if (r > cap) r = cap;
-        return r < 1 ? (int64_t)1 : r;
-    };
-    const int64_t r128 = ranges(t128), r64 = ranges(t64);
-    if (t128 * r128 * 2 < slots) return {64, (int)r64, 1};
-    return {128, (int)r128, 1};
-}
-// The plan with the least modelled time, of those with at most max_ranges ranges.  The model is measured (22 products of this
-// file's kinds, [258 .. 7520] x [100 .. 7520] over [100 .. 7520], some 380 plans; what it picks is within 1 % of the best of
-// them on average, 3 % at most): a stage of a group takes `chain` us when it has the compute unit to itself, the groups that
-// share a unit take `unit` us of its throughput each, a launch `base` us and every further round of blocks 2.6; outputs leave at 4.8 TB/s; adding ranges up is one more
-// launch, whose 14 TB/s say that the partial matrices come back out of the caches.  Blocks that run on a unit at a time: what
-// registers and LDS leave room for.
-static FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int max_ranges, bool groups4)
-{
-    struct Kind {
-        int bm, groups, resident;
-        double chain, unit, base;
-    };
-    static const Kind kinds[] = {{128, 1, 3, 0.51, 0.36, 5.4}, {128, 2, 1, 0.51, 0.36, 5.4}, {64, 1, 4, 0.46, 0.26, 3.7},
-                                 {64, 2, 2, 0.46, 0.26, 3.7},  {64, 4, 1, 0.46, 0.26, 3.7}};
-    const bool split = f32_split_mode() != 0;
-    const double out_mb = (double)M * N * 4e-6;
-    FgPlan best = {128, 1, 1};
-    double best_us = 1e30;
-    for (const Kind &kd : kinds) {
-        if (kd.groups > 1 && (!split || (kd.groups == 4 && !groups4))) continue;
-        const int64_t tiles = cdiv(M, kd.bm) * cdiv(N, FG_BN);
-        for (int r = 1; r <= max_ranges; ++r) {
-            const int64_t chunk = cdiv(cdiv(K, r), FG_BK) * FG_BK;
-            if (r > 1 && (cdiv(K, chunk) != r || chunk < 64)) continue;   // every range holds something, and four stages at least
-            const int64_t per_cu = cdiv(tiles * r, num_cus), stages = cdiv(chunk / FG_BK, kd.groups);
-            const int64_t rounds = cdiv(per_cu, kd.resident);
-            const double us = kd.base + 2.6 * (rounds - 1) + stages * (rounds * kd.chain + per_cu * kd.groups * kd.unit) + out_mb * r * 0.21 +
-                              (r > 1 ? 4.2 + out_mb * r * 0.07 : 0.0);
-            if (us < best_us) {
-                best_us = us;
-                best = {kd.bm, r, kd.groups};
-            }
-        }
-    }
-    return best;
-}
 // z = x . N^T and t = dy . C, [tokens x k] over K = in_f or out_f; dC = dy^T . z, [out_f x k] over the tokens: ranges there is room for
 static int zt_room(const rdb_linear_desc *d, int64_t K, int num_cus) { return fg_room(d->tokens, d->k, K, num_cus, 128, 32).ranges; }
 static int dc_room(const rdb_linear_desc *d, int num_cus) { return fg_room(d->out_f, d->k, d->tokens, num_cus, 256, 64).ranges; }
@@ -665,134 +101,6 @@ int64_t linear_f32_workspace(int op, const rdb_linear_desc *d, int num_cus)
     const int r = dc_room(d, num_cus);
     // ... and, for the gradient of the random bias's scale, one value per 64 x 128 tile of [tokens x out_f]
     return with_parts(d->in_f) + (r > 1 ? (int64_t)r * up256(d->out_f * d->k * 4) : 0) + up256(cdiv(d->tokens, 64) * cdiv(d->out_f, FG_BN) * 4);
-}
-
-struct FgProduct {
-    const float *a;
-    int64_t lda, a_elems;
-    const float *b;
-    int64_t ldb, b_elems;
-    float *out;
-    int64_t ldo;
-    const float *bias;
-    int64_t M, N, K;
-    int bm;                 // tile height: 128 or 64; 0: fg_launch plans it, and the groups
-    int groups;             // per block: 1, 2 or (64-row tiles) 4
-    int64_t kchunk;         // contraction values per range (a multiple of FG_BK); 0: one range
-    int64_t split_stride;   // floats between the ranges' outputs
-    uint32_t seed;
-    // the random-bias products (FG_NOISE_1D on the B side): index steps, and what the epilogue does
-    uint32_t nsR, nsK;
-    const float *scale;     // out += scale[0] * product
-    const float *dotm;      // or: dot_part[block] = <product tile, dotm tile>
-    int64_t lddot;
-    float *dot_part;
-    // bytes per element of the A and B matrices (2: bf16), and whether out / bias / dotm and scale are bf16
-    int a_es = 4, b_es = 4, out_bf16 = 0, scale_bf16 = 0;
-    // the products as six bf16 matrix instructions on three-way splits of the operands (fg_split3); materialising stays on the
-    // fp32 matrix instructions (its unit-coefficient results are compared bit for bit)
-    bool split = f32_split_mode() != 0;
-};
-
-#define FG_LAUNCH_GROUPS(BM_, G_, EPI_)                                                                               \
-    do {                                                                                                            \
-        const int nt = FG_THREADS * G_;                                                                             \
-        if (any16) {                                                                                                \
-            if (vec) f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, true, true, true><<<grid, nt, 0, s>>>(p);           \
-            else f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, false, true, true><<<grid, nt, 0, s>>>(p);              \
-        } else {                                                                                                    \
-            if (vec) f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, true, true><<<grid, nt, 0, s>>>(p);                 \
-            else f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, false, true><<<grid, nt, 0, s>>>(p);                    \
-        }                                                                                                           \
-    } while (0)
-#define FG_LAUNCH(BM_, EPI_)                                                                                        \
-    do {                                                                                                            \
-        if (q.split) FG_LAUNCH_GROUPS(BM_, 1, EPI_);                                                                \
-        else if (vec) f32_gemm_kernel<BM_, 1, ASRC, BSRC, EPI_, true><<<grid, FG_THREADS, 0, s>>>(p);               \
-        else f32_gemm_kernel<BM_, 1, ASRC, BSRC, EPI_, false><<<grid, FG_THREADS, 0, s>>>(p);                       \
-    } while (0)
-// The kernels with several groups per block, and whether there is one: four groups' buffers do not fit in LDS where a side is read
-// across its rows (its planes are padded), and only the plain epilogues are built.
-template <int ASRC, int BSRC> struct FgGroups {
-    static constexpr bool any = BSRC != FG_NOISE_1D, four = any && ASRC != FG_MCONT && BSRC != FG_MCONT;
-};
-template <int ASRC, int BSRC> static int fg_launch(FgProduct q, int num_cus, hipStream_t s, const char *name)
-{
-    typedef FgGroups<ASRC, BSRC> Groups;
-    if (!q.bm) {
-        const bool plain = Groups::any && !q.scale;
-        const FgPlan pl = plain ? fg_plan(q.M, q.N, q.K, num_cus, 1, Groups::four) : fg_room(q.M, q.N, q.K, num_cus, q.K, 1);
-        q.bm = pl.bm;
-        q.groups = pl.groups;
-    }
-    if (q.a_elems >= (1ll << 29) || q.b_elems >= (1ll << 29) || q.M >= (1ll << 30) || q.N >= (1ll << 30) || q.K >= (1ll << 30)) return RDB_E_UNSUPPORTED;
-    FgParams p = {};
-    p.a = q.a;
-    p.lda = q.lda;
-    p.b = q.b;
-    p.ldb = q.ldb;
-    p.out = q.out;
-    p.ldo = q.ldo;
-    p.split_stride = q.split_stride;
-    p.bias = q.bias;
-    p.M = (int)q.M;
-    p.N = (int)q.N;
-    p.K = (int)q.K;
-    p.kchunk = (int)(q.kchunk > 0 ? q.kchunk : cdiv(q.K, FG_BK) * FG_BK);
-    p.a_bytes = q.a_elems * q.a_es;
-    p.b_bytes = q.b_elems * q.b_es;
-    p.a_es = q.a_es;
-    p.b_es = q.b_es;
-    p.out_bf16 = q.out_bf16;
-    p.scale_bf16 = q.scale_bf16;
-    p.seed = q.seed;
-    p.nsR = q.nsR;
-    p.nsK = q.nsK;
-    p.scale = q.scale;
-    p.dotm = q.dotm;
-    p.lddot = q.lddot;
-    p.dot_part = q.dot_part;
-    const int splits = (int)cdiv(q.K, p.kchunk);
-    // 16-byte pieces when both matrices allow them: aligned bases and leading dimensions, and the extent along a piece a multiple of 4
-    // (along the rows of a matrix: the contraction; across them: the rows of the tile)
-    auto vec_ok = [&](int src, const float *m, int64_t ld, int64_t rows) {
-        if (src != FG_KCONT && src != FG_MCONT) return true;
-        return fg_aligned16(m) && ld % 4 == 0 && (src == FG_KCONT ? q.K % 4 == 0 : rows % 4 == 0);
-    };
-    const bool vec = vec_ok(ASRC, q.a, q.lda, q.M) && vec_ok(BSRC, q.b, q.ldb, q.N);   // bf16 matrices: 8-byte pieces of four values
-    const bool any16 = q.a_es == 2 || ((BSRC == FG_KCONT || BSRC == FG_MCONT) && q.b_es == 2);   // the A side is always a matrix
-    if (cdiv(q.N, FG_BN) > 65535) return RDB_E_UNSUPPORTED;   // the grid's y
-    const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)splits);
-    if constexpr (BSRC == FG_NOISE_1D) {   // the random-bias products: added on top of an output, or reduced against a matrix
-        if (q.bm == 128) {
-            if (q.dotm) FG_LAUNCH(128, FG_DOT);
-            else FG_LAUNCH(128, FG_ADD_SCALED);
-        } else {
-            if (q.dotm) FG_LAUNCH(64, FG_DOT);
-            else FG_LAUNCH(64, FG_ADD_SCALED);
-        }
-    } else if (q.scale) {        // materialising W with its random-bias share
-        if (q.bm == 128) FG_LAUNCH(128, FG_STORE_RBIAS);
-        else FG_LAUNCH(64, FG_STORE_RBIAS);
-    } else if (q.bm == 128 && q.groups == 2) {
-        if (q.bias) FG_LAUNCH_GROUPS(128, 2, FG_STORE_BIAS);
-        else FG_LAUNCH_GROUPS(128, 2, FG_STORE);
-    } else if (q.bm == 128) {
-        if (q.bias) FG_LAUNCH(128, FG_STORE_BIAS);
-        else FG_LAUNCH(128, FG_STORE);
-    } else if (q.groups == 2) {
-        if (q.bias) FG_LAUNCH_GROUPS(64, 2, FG_STORE_BIAS);
-        else FG_LAUNCH_GROUPS(64, 2, FG_STORE);
-    } else if (q.groups == 4) {
-        if constexpr (Groups::four) {
-            if (q.bias) FG_LAUNCH_GROUPS(64, 4, FG_STORE_BIAS);
-            else FG_LAUNCH_GROUPS(64, 4, FG_STORE);
-        }
-    } else {
-        if (q.bias) FG_LAUNCH(64, FG_STORE_BIAS);
-        else FG_LAUNCH(64, FG_STORE);
-    }
-    return check_launch(name);
 }
 
 static bool fg_ws_ok(int op, const rdb_linear_desc *d, int num_cus, const void *ws, int64_t bytes)
@@ -1072,4 +380,42 @@ int coef_grad_mat_f32(float *dcoef, const void *dW, int dw_dtype, int64_t coef_r
                                                   s, "f32_gemm_kernel (dcoef = dW . N^T)");
 }
 
+// ----------------------------------------------------------------------------------------------- a dense product
+static int product_room(int64_t M, int64_t N, int64_t K, int num_cus) { return fg_room(M, N, K, num_cus, 256, 64).ranges; }
+static bool product_ok(int64_t M, int64_t N, int64_t K) { return M > 0 && N > 0 && K > 0 && M * N < (1ll << 29) && K < (1 << 30); }
+
 }  // namespace rdb
+
+using namespace rdb;
+
+extern "C" int64_t rdb_product_f32_workspace_bytes(int64_t M, int64_t N, int64_t K)
+{
+    if (!product_ok(M, N, K)) return 0;
+    const int r = product_room(M, N, K, num_compute_units());
+    return r > 1 ? (int64_t)r * up256(M * N * 4) : 0;
+}
+
+extern "C" int rdb_product_f32(float *out, const float *a, int64_t lda, int a_across, const float *b, int64_t ldb, int b_across, const float *bias, int64_t M,
+                               int64_t N, int64_t K, void *workspace, int64_t workspace_bytes, void *stream)
+{
+    if (M < 0 || N < 0 || K < 0) return set_error(RDB_E_SHAPE, "rdb_product_f32: negative size %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
+    if (!product_ok(M, N, K) || (a_across && !b_across))
+        return set_error(RDB_E_UNSUPPORTED, "rdb_product_f32: needs non-empty sizes, M * N below 2^29 and not (a_across without b_across)");
+    if (!out || !a || !b) return set_error(RDB_E_NULL, "rdb_product_f32: out, a or b is NULL");
+    if (lda < (a_across ? M : K) || ldb < (b_across ? N : K)) return set_error(RDB_E_SHAPE, "rdb_product_f32: leading dimension smaller than the row");
+    if (lda * (a_across ? K : M) >= (1ll << 29) || ldb * (b_across ? K : N) >= (1ll << 29))
+        return set_error(RDB_E_UNSUPPORTED, "rdb_product_f32: matrices of less than 2^29 elements");
+    const int num_cus = num_compute_units();
+    FgProduct q = {a, lda, a_across ? (K - 1) * lda + M : (M - 1) * lda + K, b, ldb, b_across ? (K - 1) * ldb + N : (N - 1) * ldb + K, out, N, bias, M, N, K,
+                   0, 0, 0, 0, 0u};
+    const int64_t stride = up256(M * N * 4);
+    int room = product_room(M, N, K, num_cus);
+    if (bias || !workspace || !fg_aligned16(workspace)) room = 1;   // the bias is added by the product's own epilogue
+    else if (room * stride > workspace_bytes) room = (int)std::max<int64_t>(1, workspace_bytes / stride);
+    float *part = static_cast<float *>(workspace);
+    hipStream_t s = (hipStream_t)stream;
+    const char *name = "f32_gemm_kernel (dense product)";
+    if (a_across) return fg_launch_ranges<FG_MCONT, FG_MCONT>(q, room, part, stride / 4, num_cus, s, name);
+    if (b_across) return fg_launch_ranges<FG_KCONT, FG_MCONT>(q, room, part, stride / 4, num_cus, s, name);
+    return fg_launch_ranges<FG_KCONT, FG_KCONT>(q, room, part, stride / 4, num_cus, s, name);
+}

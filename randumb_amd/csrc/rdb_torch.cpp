@@ -110,13 +110,87 @@ rdb_linear_desc desc(const Tensor &rows, const Layer &l, const Tensor &c)
     return desc(rows.size(0), l, c.size(-1), c.dim() == 1 ? 0 : c.size(0), rows.scalar_type(), c.scalar_type());
 }
 
+// ----------------------------------------------------------------------------------------------- pseudorandom vectors and biases
+// n values of a contiguous vector-coef tensor, b[o] = sum_m noise(PRIME*o + m) coef[m] (+ s noise1d(o)), in the coefficients' dtype
+Tensor coef_values(const Tensor &coef, const OptTensor &scale_bias, int64_t n, int64_t seed)
+{
+    const Tensor c = native(coef), sb = scale_bias && scale_bias->defined() ? native(*scale_bias).to(c.scalar_type()) : Tensor();
+    const c10::OptionalDeviceGuard guard(c.device());
+    Tensor out = at::empty({n}, c.options().dtype(at::kFloat));
+    check(rdb_materialize_fwd(out.data_ptr<float>(), c.data_ptr(), code(c.scalar_type()), 0, c.numel(), 0, 1, n, 0, 1, (uint32_t)seed, ptr(sb), stream_of(c)),
+          "rdb_materialize_fwd");
+    return out.to(coef.scalar_type());
+}
+// ... and the adjoint: fp32 gradients of coef (k values) and s from the gradient of the values
+std::pair<Tensor, Tensor> coef_grads(const Tensor &grad, int64_t k, int64_t seed, bool want_coef, bool want_scale)
+{
+    const Tensor d = native(grad);
+    const c10::OptionalDeviceGuard guard(d.device());
+    const auto f32 = d.options().dtype(at::kFloat);
+    Tensor dc, ds;
+    if (want_coef) {
+        const int64_t need = rdb_materialize_bwd_workspace_bytes(0, k, 0, d.numel());
+        const Tensor ws = bytes(need, d);
+        dc = at::empty({k}, f32);
+        check(rdb_materialize_bwd(dc.data_ptr<float>(), d.data_ptr(), code(d.scalar_type()), 0, k, 0, d.numel(), (uint32_t)seed, ptr(ws), need, stream_of(d)),
+              "rdb_materialize_bwd");
+    }
+    if (want_scale) {
+        const int64_t need = rdb_scale_bias_bwd_workspace_bytes(d.numel());
+        const Tensor ws = bytes(need, d);
+        ds = at::empty({1}, f32);
+        check(rdb_scale_bias_bwd(ds.data_ptr<float>(), d.data_ptr(), code(d.scalar_type()), d.numel(), (uint32_t)seed, ptr(ws), need, stream_of(d)),
+              "rdb_scale_bias_bwd");
+    }
+    return {dc, ds};
+}
+
+// A layer's bias: a dense vector (seed < 0), or a pseudorandom one given by its coefficients (and, with a fused random bias, its scale)
+struct Bias {
+    OptTensor coef, scale;
+    int64_t seed = -1;
+    explicit operator bool() const { return coef.has_value(); }
+    int tensors() const { return (coef ? 1 : 0) + (scale ? 1 : 0); }
+    Tensor values(int64_t n, at::ScalarType dtype) const
+    {
+        if (!coef) return Tensor();
+        return (seed < 0 ? *coef : coef_values(*coef, scale, n, seed)).to(dtype).contiguous();
+    }
+    // what its gradient needs of it: whether there is one, length, seed, dtypes
+    std::vector<int64_t> meta() const
+    {
+        return {coef ? coef->numel() : -1, seed, coef ? (int64_t)coef->scalar_type() : 0, scale ? (int64_t)scale->scalar_type() : -1};
+    }
+};
+// (gradient of the bias or its coefficients, gradient of its scale) from the column sums of dy; `at` is the bias's index among the
+// function's tensor inputs
+std::pair<Tensor, Tensor> bias_grads(AutogradContext *ctx, const Tensor &dy0, const std::vector<int64_t> &m, int at)
+{
+    if (m[0] < 0) return {};
+    const bool want_c = ctx->needs_input_grad(at), want_s = m[3] >= 0 && ctx->needs_input_grad(at + 1);
+    if (!want_c && !want_s) return {};
+    if (m[1] < 0) return {dy0.sum(0).to((at::ScalarType)m[2]), Tensor()};
+    const Tensor dy = act(dy0);
+    const auto f32 = dy.options().dtype(at::kFloat);
+    Tensor dc = want_c ? at::empty({m[0]}, f32) : Tensor(), ds = want_s ? at::empty({1}, f32) : Tensor();
+    const int64_t need = rdb_bias_bwd_workspace_bytes(dy.size(0), dy.size(1));
+    const Tensor ws = bytes(need, dy);
+    const c10::OptionalDeviceGuard guard(dy.device());
+    check(rdb_bias_bwd(want_c ? dc.data_ptr<float>() : nullptr, want_s ? ds.data_ptr<float>() : nullptr, dy.data_ptr(), code(dy.scalar_type()), dy.stride(0),
+                       dy.size(0), dy.size(1), m[0], (uint32_t)m[1], ptr(ws), need, stream_of(dy)),
+          "rdb_bias_bwd");
+    if (want_c) dc = dc.to((at::ScalarType)m[2]);
+    if (want_s) ds = ds.to((at::ScalarType)m[3]);
+    return {dc, ds};
+}
+
 // ----------------------------------------------------------------------------------------------- the library's calls
-Tensor linear_fwd(const Tensor &x0, const Tensor &coefs, const Layer &l, const OptTensor &scale_bias, const OptTensor &bias)
+Tensor linear_fwd(const Tensor &x0, const Tensor &coefs, const Layer &l, const OptTensor &scale_bias, const Bias &bias)
 {
     const Tensor x = act(x0), c = native(coefs);
     const Tensor sb = scale_bias ? native(*scale_bias).to(c.scalar_type()) : Tensor();
-    const Tensor b = bias ? bias->to(x.scalar_type()).contiguous() : Tensor();
     const c10::OptionalDeviceGuard guard(x.device());
+    const Tensor b = bias.values(l.out_f, x.scalar_type());
     Tensor y = at::empty({x.size(0), l.out_f}, x.options());
     const rdb_linear_desc d = desc(x, l, c);
     const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_FWD, &d);
@@ -178,19 +252,18 @@ std::pair<Tensor, Tensor> linear_bwd_dcoef(const Tensor &dy0, const Tensor &x0, 
 
 rdb_linear_desc rbias_desc(const Tensor &rows, const Layer &l) { return desc(rows.size(0), l, 8, l.out_f, at::kBFloat16, at::kBFloat16); }
 
-// dbias: the column sums of dy
-Tensor bias_grad(const Tensor &dy, at::ScalarType dtype) { return dy.sum(0).to(dtype); }
-
 // ----------------------------------------------------------------------------------------------- one-call form
 // y = x.W^T (+ bias) with x saved; the three products of the layer as three calls.
 class OneCallLinear : public Function<OneCallLinear> {
   public:
-    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &coefs, const OptTensor &scale_bias, const OptTensor &bias, const Layer &l)
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &coefs, const OptTensor &scale_bias, const OptTensor &bias,
+                          const OptTensor &bias_scale, int64_t bias_seed, const Layer &l)
     {
+        const Bias b{bias, bias_scale, bias_seed};
         ctx->save_for_backward({x, coefs, scale_bias.value_or(Tensor())});
-        ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, l.sO, l.sI, (int64_t)l.seed, scale_bias ? 1 : 0,
-                                                        bias ? (int64_t)bias->scalar_type() : -1};
-        return linear_fwd(x, coefs, l, scale_bias, bias);
+        ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, l.sO, l.sI, (int64_t)l.seed, scale_bias ? 1 : 0};
+        ctx->saved_data["bias"] = b.meta();
+        return linear_fwd(x, coefs, l, scale_bias, b);
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
@@ -198,13 +271,12 @@ class OneCallLinear : public Function<OneCallLinear> {
         const Tensor &x = saved[0], &coefs = saved[1], &sb = saved[2];
         const auto m = ctx->saved_data["layer"].toIntVector();
         const Layer l{m[0], m[1], m[2], m[3], (uint32_t)m[4]};
-        const bool has_sb = m[5] != 0, has_bias = m[6] >= 0;
+        const bool has_sb = m[5] != 0;
         const at::AutoGradMode no_grad(false);
         const bool want_dx = ctx->needs_input_grad(0), want_dc = ctx->needs_input_grad(1);
         bool want_sb = has_sb && ctx->needs_input_grad(2);
-        const bool want_b = has_bias && ctx->needs_input_grad(has_sb ? 3 : 2);
         const Tensor dy = grads[0].contiguous();
-        Tensor dx, dc, dsb, db;
+        Tensor dx, dc, dsb;
         if (want_dx && want_sb && l.sO == l.in_f && l.sI == 1) {
             // the random-bias product dy.R that dx needs anyway also gives the gradient of the bias's scale (reduced against x
             // in the same pass), so the coefficient gradient below comes from the factored kernels and dW is never formed
@@ -221,8 +293,8 @@ class OneCallLinear : public Function<OneCallLinear> {
             dc = both.first.to(coefs.scalar_type());
             if (want_sb) dsb = both.second.to(sb.scalar_type());
         }
-        if (want_b) db = bias_grad(dy, (at::ScalarType)m[6]);
-        return {dx, dc, dsb, db, Tensor()};
+        const auto db = bias_grads(ctx, dy, ctx->saved_data["bias"].toIntVector(), has_sb ? 3 : 2);
+        return {dx, dc, dsb, db.first, db.second, Tensor(), Tensor()};
     }
 };
 
@@ -231,14 +303,16 @@ class OneCallLinear : public Function<OneCallLinear> {
 // of x; with the fused random bias its full-rank share is added on top in both directions and x is saved as well.
 class ProjectedLinear : public Function<ProjectedLinear> {
   public:
-    static Tensor forward(AutogradContext *ctx, const Tensor &x0, const Tensor &coefs, const OptTensor &bias, const OptTensor &scale_bias, const Layer &l)
+    static Tensor forward(AutogradContext *ctx, const Tensor &x0, const Tensor &coefs, const OptTensor &bias, const OptTensor &bias_scale, int64_t bias_seed,
+                          const OptTensor &scale_bias, const Layer &l)
     {
+        const Bias pb{bias, bias_scale, bias_seed};
         const Tensor x = act(x0), c = coefs.contiguous();
         const c10::OptionalDeviceGuard guard(x.device());
         const rdb_linear_desc d = desc(x, l, c);
         const int64_t need = rdb_linear_projection_bytes(&d);
         Tensor state = bytes(need, x), y = at::empty({x.size(0), l.out_f}, x.options());
-        const Tensor b = bias ? bias->to(x.scalar_type()).contiguous() : Tensor();
+        const Tensor b = pb.values(l.out_f, x.scalar_type());
         void *s = stream_of(x);
         check(rdb_linear_project_fwd(y.data_ptr(), l.out_f, ptr(state), x.data_ptr(), x.stride(0), c.data_ptr(), ptr(b), &d, s), "rdb_linear_project_fwd");
         if (scale_bias) {
@@ -248,7 +322,8 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         }
         tick(x);
         ctx->save_for_backward({state, coefs, scale_bias.value_or(Tensor()), scale_bias ? x0 : Tensor()});
-        ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, (int64_t)l.seed, scale_bias ? 1 : 0, bias ? (int64_t)bias->scalar_type() : -1};
+        ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, (int64_t)l.seed, scale_bias ? 1 : 0, pb.tensors()};
+        ctx->saved_data["bias"] = pb.meta();
         return y;
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
@@ -257,10 +332,9 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         const Tensor &state = saved[0], &coefs = saved[1], &scale_bias = saved[2];
         const auto m = ctx->saved_data["layer"].toIntVector();
         const Layer l{m[0], m[1], m[0], 1, (uint32_t)m[2]};
-        const bool has_sb = m[3] != 0, has_bias = m[4] >= 0;
+        const bool has_sb = m[3] != 0;
         const at::AutoGradMode no_grad(false);
-        const bool want_x = ctx->needs_input_grad(0), want_dc = ctx->needs_input_grad(1);
-        const bool want_b = has_bias && ctx->needs_input_grad(2), want_sb = has_sb && ctx->needs_input_grad(has_bias ? 3 : 2);
+        const bool want_x = ctx->needs_input_grad(0), want_dc = ctx->needs_input_grad(1), want_sb = has_sb && ctx->needs_input_grad(2 + m[4]);
         const bool want_dx = want_x || want_sb;   // the gradient of the scale comes out of the random-bias share of dx
         Tensor dy = act(grads[0]);
         const bool f32 = coefs.scalar_type() == at::kFloat;
@@ -269,7 +343,7 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         const c10::OptionalDeviceGuard guard(dy.device());
         const rdb_linear_desc d = desc(dy, l, c);
         void *s = stream_of(dy);
-        Tensor dx, dc, dsb, db;
+        Tensor dx, dc, dsb;
         if (want_dc && (want_dx || f32)) {
             // bf16 coefficients: their gradient leaves the kernel that adds it up in bf16, where the layer runs as one chunk of tokens
             const bool to_bf16 = !f32 && rdb_linear_projection_chunks(&d, nullptr) == 1;
@@ -307,55 +381,173 @@ class ProjectedLinear : public Function<ProjectedLinear> {
             }
         }
         if (!want_x) dx = Tensor();
-        if (want_b) db = bias_grad(dy, (at::ScalarType)m[4]);
-        return {dx, dc, db, dsb, Tensor()};
+        const auto db = bias_grads(ctx, dy, ctx->saved_data["bias"].toIntVector(), 2);
+        return {dx, dc, db.first, db.second, Tensor(), dsb, Tensor()};
     }
 };
 
-// ----------------------------------------------------------------------------------------------- a pseudorandom vector (a layer's bias)
-// b[o] = sum_m noise(PRIME*o + m) coef[m] (+ s noise1d(o)), in the coefficients' dtype, and the gradients of coef and s.
-class VectorFromCoefs : public Function<VectorFromCoefs> {
+// ----------------------------------------------------------------------------------------------- the vector-coef layer
+// Gradient of the values of a vector-coef tensor -> gradients of its coefficients and scale, differentiable (for create_graph).
+class CoefGrads : public Function<CoefGrads> {
   public:
-    static Tensor forward(AutogradContext *ctx, const Tensor &coef, const OptTensor &scale_bias, int64_t n, int64_t seed)
+    static variable_list forward(AutogradContext *ctx, const Tensor &dvalues, int64_t k, int64_t seed, bool want_scale)
     {
-        ctx->saved_data["vector"] = std::vector<int64_t>{coef.numel(), seed, (int64_t)coef.scalar_type(), scale_bias ? (int64_t)scale_bias->scalar_type() : -1};
-        return values(coef, scale_bias, n, seed);
-    }
-    static Tensor values(const Tensor &coef, const OptTensor &scale_bias, int64_t n, int64_t seed)
-    {
-        const Tensor c = native(coef), sb = scale_bias ? native(*scale_bias).to(c.scalar_type()) : Tensor();
-        const c10::OptionalDeviceGuard guard(c.device());
-        Tensor out = at::empty({n}, c.options().dtype(at::kFloat));
-        check(rdb_materialize_fwd(out.data_ptr<float>(), c.data_ptr(), code(c.scalar_type()), 0, c.numel(), 0, 1, n, 0, 1, (uint32_t)seed, ptr(sb), stream_of(c)),
-              "rdb_materialize_fwd");
-        return out.to(coef.scalar_type());
+        ctx->saved_data["n"] = dvalues.numel();
+        ctx->saved_data["seed"] = seed;
+        ctx->saved_data["dtype"] = (int64_t)dvalues.scalar_type();
+        ctx->saved_data["sizes"] = dvalues.sizes().vec();
+        const auto g = coef_grads(dvalues, k, seed, true, want_scale);
+        return want_scale ? variable_list{g.first, g.second} : variable_list{g.first};
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
-        const auto m = ctx->saved_data["vector"].toIntVector();
+        const at::AutoGradMode no_grad(false);
+        const Tensor v = coef_values(grads[0], grads.size() > 1 ? OptTensor(grads[1]) : OptTensor(), ctx->saved_data["n"].toInt(), ctx->saved_data["seed"].toInt());
+        return {v.to((at::ScalarType)ctx->saved_data["dtype"].toInt()).view(ctx->saved_data["sizes"].toIntVector()), Tensor(), Tensor(), Tensor()};
+    }
+};
+// The values themselves, differentiable in coef and scale.
+class CoefValues : public Function<CoefValues> {
+  public:
+    static Tensor forward(AutogradContext *ctx, const Tensor &coef, const OptTensor &scale_bias, int64_t n, int64_t seed)
+    {
+        ctx->saved_data["m"] = std::vector<int64_t>{coef.numel(), seed, (int64_t)coef.scalar_type(), scale_bias ? (int64_t)scale_bias->scalar_type() : -1};
+        return coef_values(coef, scale_bias, n, seed);
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const auto m = ctx->saved_data["m"].toIntVector();
+        const auto g = CoefGrads::apply(grads[0].contiguous(), m[0], m[1], m[3] >= 0);
+        return {g[0].to((at::ScalarType)m[2]), m[3] >= 0 ? g[1].to((at::ScalarType)m[3]) : Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// out [M x N] = A . B^T (+ bias); A [M x K], B [N x K], or stored transposed (across).  fp32: the library's own product; bf16: torch's
+Tensor product(const Tensor &a, bool a_across, const Tensor &b, bool b_across, const Tensor &bias)
+{
+    const int64_t M = a.size(a_across ? 1 : 0), K = a.size(a_across ? 0 : 1), N = b.size(b_across ? 1 : 0);
+    if (a.scalar_type() == at::kFloat) {
+        Tensor out = at::empty({M, N}, a.options());
+        const int64_t need = rdb_product_f32_workspace_bytes(M, N, K);
+        const Tensor ws = bytes(need, a);
+        const int rc = rdb_product_f32(out.data_ptr<float>(), a.data_ptr<float>(), a.stride(0), a_across, b.data_ptr<float>(), b.stride(0), b_across,
+                                       bias.defined() ? bias.data_ptr<float>() : nullptr, M, N, K, ptr(ws), need, stream_of(a));
+        if (rc != RDB_E_UNSUPPORTED) {
+            check(rc, "rdb_product_f32");
+            return out;
+        }
+    }
+    const Tensor l = a_across ? a.t() : a, r = b_across ? b : b.t();
+    return bias.defined() ? at::addmm(bias, l, r) : at::mm(l, r);
+}
+
+// y = x.W^T (+ b) with W and b vector-coef tensors: W is formed (k hashed values per element), multiplied as a dense matrix, and
+// in the backward pass dW = dy^T.x is formed and contracted with the hashed values.  Forming W is the most expensive step of the
+// layer, and the backward pass needs it again for dx: it is kept for that where it takes no more memory than the activations x
+// and y of this pass, which the program holds anyway; otherwise it is formed again, so that a layer never holds more than twice
+// what its activations take (1024 tokens x 768 -> 3072, k = 256: 9.4 MB beside 15.7 MB).
+class VectorLinear : public Function<VectorLinear> {
+  public:
+    static Tensor forward(AutogradContext *ctx, const Tensor &x0, const Tensor &coef, const OptTensor &scale, const OptTensor &bias, const OptTensor &bias_scale,
+                          int64_t bias_seed, const Layer &l)
+    {
+        const Bias b{bias, bias_scale, bias_seed};
+        const c10::OptionalDeviceGuard guard(x0.device());
+        const Tensor W = coef_values(coef, scale, l.out_f * l.in_f, l.seed).view({l.out_f, l.in_f});
+        Tensor y = values(x0, W, b, l);
+        const bool keep = ctx != nullptr && W.numel() <= x0.numel() + y.numel();
+        if (ctx) {
+            ctx->save_for_backward({x0, coef, scale.value_or(Tensor()), keep && x0.requires_grad() ? W : Tensor()});
+            ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, (int64_t)l.seed, scale ? (int64_t)scale->scalar_type() : -1};
+            ctx->saved_data["bias"] = b.meta();
+        }
+        return y;
+    }
+    static Tensor values(const Tensor &x0, const Tensor &W, const Bias &b, const Layer &l)
+    {
+        auto sizes = x0.sizes().vec();
+        sizes.back() = l.out_f;
+        return product(act(x0.reshape({-1, l.in_f})), false, W, false, b.values(l.out_f, x0.scalar_type())).view(sizes);
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const auto m = ctx->saved_data["layer"].toIntVector();
+        const Layer l{m[0], m[1], m[0], 1, (uint32_t)m[2]};
+        const bool has_scale = m[3] >= 0;
+        const bool want_x = ctx->needs_input_grad(0), want_c = ctx->needs_input_grad(1), want_s = has_scale && ctx->needs_input_grad(2);
+        const Tensor &x0 = saved[0], &coef = saved[1];
+        const OptTensor scale = has_scale ? OptTensor(saved[2]) : OptTensor();
+        const c10::OptionalDeviceGuard guard(x0.device());
+        Tensor dx, dc, ds;
+        const Tensor dy = act(grads[0].reshape({-1, l.out_f}));
+        if (at::GradMode::is_enabled()) {   // create_graph: the same products from differentiable operators
+            const Tensor x = x0.reshape({-1, l.in_f});
+            if (want_x) dx = dy.mm(CoefValues::apply(coef, scale, l.out_f * l.in_f, (int64_t)l.seed).view({l.out_f, l.in_f})).view(x0.sizes());
+            if (want_c || want_s) {
+                const auto g = CoefGrads::apply(dy.t().mm(x), coef.numel(), (int64_t)l.seed, want_s);
+                if (want_c) dc = g[0].to(coef.scalar_type());
+                if (want_s) ds = g[1].to((at::ScalarType)m[3]);
+            }
+            const auto bm = ctx->saved_data["bias"].toIntVector();
+            if (bm[0] < 0) return {dx, dc, ds, Tensor(), Tensor(), Tensor(), Tensor()};
+            const Tensor db = dy.sum(0);
+            if (bm[1] < 0) return {dx, dc, ds, db.to((at::ScalarType)bm[2]), Tensor(), Tensor(), Tensor()};
+            const auto g = CoefGrads::apply(db, bm[0], bm[1], bm[3] >= 0);
+            return {dx, dc, ds, g[0].to((at::ScalarType)bm[2]), bm[3] >= 0 ? g[1].to((at::ScalarType)bm[3]) : Tensor(), Tensor(), Tensor()};
+        }
+        if (want_x) {
+            const Tensor W = saved[3].defined() ? saved[3] : coef_values(coef, scale, l.out_f * l.in_f, l.seed).view({l.out_f, l.in_f});
+            dx = product(dy, false, W, true, Tensor()).view(x0.sizes());
+        }
+        if (want_c || want_s) {
+            const auto g = coef_grads(product(dy, true, act(x0.reshape({-1, l.in_f})), true, Tensor()), coef.numel(), l.seed, want_c, want_s);
+            if (want_c) dc = g.first.to(coef.scalar_type());
+            if (want_s) ds = g.second.to((at::ScalarType)m[3]);
+        }
+        const auto db = bias_grads(ctx, dy, ctx->saved_data["bias"].toIntVector(), has_scale ? 3 : 2);
+        return {dx, dc, ds, db.first, db.second, Tensor(), Tensor()};
+    }
+};
+
+// rows idx of a (*, rowsize) vector-coef table, fp32
+class EmbedRows : public Function<EmbedRows> {
+  public:
+    static Tensor forward(AutogradContext *ctx, const Tensor &idx0, const Tensor &coef, int64_t rowsize, int64_t seed)
+    {
+        const Tensor idx = idx0.to(at::kLong).contiguous();
+        if (ctx) {
+            ctx->save_for_backward({idx});
+            ctx->saved_data["m"] = std::vector<int64_t>{coef.numel(), rowsize, seed, (int64_t)coef.scalar_type()};
+        }
+        return rows(idx, coef, rowsize, seed);
+    }
+    static Tensor rows(const Tensor &idx, const Tensor &coef, int64_t rowsize, int64_t seed)
+    {
+        const Tensor c = native(coef);
+        const c10::OptionalDeviceGuard guard(c.device());
+        auto sizes = idx.sizes().vec();
+        sizes.push_back(rowsize);
+        Tensor out = at::empty(sizes, c.options().dtype(at::kFloat));
+        check(rdb_embed_fwd(out.data_ptr<float>(), idx.data_ptr<int64_t>(), idx.numel(), c.data_ptr(), code(c.scalar_type()), c.numel(), rowsize, (uint32_t)seed,
+                            stream_of(c)),
+              "rdb_embed_fwd");
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const Tensor idx = ctx->get_saved_variables()[0];
+        const auto m = ctx->saved_data["m"].toIntVector();
         const at::AutoGradMode no_grad(false);
         const Tensor d = native(grads[0]);
         const c10::OptionalDeviceGuard guard(d.device());
-        const auto f32 = d.options().dtype(at::kFloat);
-        Tensor dc, ds;
-        if (ctx->needs_input_grad(0)) {
-            const int64_t need = rdb_materialize_bwd_workspace_bytes(0, m[0], 0, d.numel());
-            const Tensor ws = bytes(need, d);
-            dc = at::empty({m[0]}, f32);
-            check(rdb_materialize_bwd(dc.data_ptr<float>(), d.data_ptr(), code(d.scalar_type()), 0, m[0], 0, d.numel(), (uint32_t)m[1], ptr(ws), need,
-                                      stream_of(d)),
-                  "rdb_materialize_bwd");
-            dc = dc.to((at::ScalarType)m[2]);
-        }
-        if (m[3] >= 0 && ctx->needs_input_grad(1)) {
-            const int64_t need = rdb_scale_bias_bwd_workspace_bytes(d.numel());
-            const Tensor ws = bytes(need, d);
-            ds = at::empty({1}, f32);
-            check(rdb_scale_bias_bwd(ds.data_ptr<float>(), d.data_ptr(), code(d.scalar_type()), d.numel(), (uint32_t)m[1], ptr(ws), need, stream_of(d)),
-                  "rdb_scale_bias_bwd");
-            ds = ds.to((at::ScalarType)m[3]);
-        }
-        return {dc, ds, Tensor(), Tensor()};
+        Tensor dc = at::empty({m[0]}, d.options().dtype(at::kFloat));
+        const int64_t need = rdb_embed_bwd_workspace_bytes(idx.numel(), m[1], m[0]);
+        const Tensor ws = bytes(need, d);
+        check(rdb_embed_bwd(dc.data_ptr<float>(), idx.data_ptr<int64_t>(), idx.numel(), d.data_ptr(), code(d.scalar_type()), m[0], m[1], (uint32_t)m[2], ptr(ws),
+                            need, stream_of(d)),
+              "rdb_embed_bwd");
+        return {Tensor(), dc.to((at::ScalarType)m[3]), Tensor(), Tensor()};
     }
 };
 
@@ -577,45 +769,73 @@ PyObject *py_takes_projected(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
 }
 
-// linear_projected(x, coefs, in_f, out_f, seed, bias, scale_bias)
-PyObject *py_linear_projected(PyObject *, PyObject *const *a, Py_ssize_t n)
+// A bias is passed as three arguments: a dense vector, None, -1; or a pseudorandom vector's coefficients, scale (or None), seed.
+Bias bias_arg(PyObject *const *a)
 {
-    return guarded([&]() -> PyObject * {
-        count_args(n, 7);
-        const Tensor &x = tensor_arg(a[0]), &c = tensor_arg(a[1]);
-        const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[2]), 1, seed_arg(a[4])};
-        const OptTensor bias = opt_arg(a[5]), sb = opt_arg(a[6]);
-        // without a backward pass to come there is no state to keep: the one-call forward
-        if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(bias) || wants_grad(sb)))
-            return THPVariable_Wrap(linear_fwd(x, c, l, sb, bias));
-        return THPVariable_Wrap(ProjectedLinear::apply(x, c, bias, sb, l));
-    });
+    Bias b{opt_arg(a[0]), opt_arg(a[1]), int_arg(a[2])};
+    if (b.seed >= (1ll << 32)) {
+        PyErr_SetString(PyExc_ValueError, "the bias's seed must fit in 32 unsigned bits");
+        throw BadArgument();
+    }
+    return b;
 }
+bool wants_grad(const Bias &b) { return wants_grad(b.coef) || wants_grad(b.scale); }
 
-// linear_one_call(x, coefs, in_f, out_f, sO, sI, seed, scale_bias, bias)
-PyObject *py_linear_one_call(PyObject *, PyObject *const *a, Py_ssize_t n)
+// linear_projected(x, coefs, in_f, out_f, seed, bias, bias_scale, bias_seed, scale_bias)
+PyObject *py_linear_projected(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
     return guarded([&]() -> PyObject * {
         count_args(n, 9);
         const Tensor &x = tensor_arg(a[0]), &c = tensor_arg(a[1]);
-        const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[4]), int_arg(a[5]), seed_arg(a[6])};
-        const OptTensor sb = opt_arg(a[7]), bias = opt_arg(a[8]);
-        if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(bias) || wants_grad(sb)))
-            return THPVariable_Wrap(linear_fwd(x, c, l, sb, bias));
-        return THPVariable_Wrap(OneCallLinear::apply(x, c, sb, bias, l));
+        const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[2]), 1, seed_arg(a[4])};
+        const Bias b = bias_arg(a + 5);
+        const OptTensor sb = opt_arg(a[8]);
+        // without a backward pass to come there is no state to keep: the one-call forward
+        if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
+            return THPVariable_Wrap(linear_fwd(x, c, l, sb, b));
+        return THPVariable_Wrap(ProjectedLinear::apply(x, c, b.coef, b.scale, b.seed, sb, l));
     });
 }
 
-// vector_from_coefs(coef, scale_bias, n, seed): a contiguous vector-coef tensor of n elements, differentiable in coef and scale_bias
-PyObject *py_vector_from_coefs(PyObject *, PyObject *const *a, Py_ssize_t n)
+// linear_one_call(x, coefs, in_f, out_f, sO, sI, seed, scale_bias, bias, bias_scale, bias_seed)
+PyObject *py_linear_one_call(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 11);
+        const Tensor &x = tensor_arg(a[0]), &c = tensor_arg(a[1]);
+        const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[4]), int_arg(a[5]), seed_arg(a[6])};
+        const OptTensor sb = opt_arg(a[7]);
+        const Bias b = bias_arg(a + 8);
+        if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
+            return THPVariable_Wrap(linear_fwd(x, c, l, sb, b));
+        return THPVariable_Wrap(OneCallLinear::apply(x, c, sb, b.coef, b.scale, b.seed, l));
+    });
+}
+
+// linear_vector(x, coef, in_f, out_f, seed, scale_bias, bias, bias_scale, bias_seed): x (..., in_f)
+PyObject *py_linear_vector(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 9);
+        const Tensor &x = tensor_arg(a[0]), &c = tensor_arg(a[1]);
+        const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[2]), 1, seed_arg(a[4])};
+        const OptTensor sb = opt_arg(a[5]);
+        const Bias b = bias_arg(a + 6);
+        if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
+            return THPVariable_Wrap(VectorLinear::forward(nullptr, x, c, sb, b.coef, b.scale, b.seed, l));
+        return THPVariable_Wrap(VectorLinear::apply(x, c, sb, b.coef, b.scale, b.seed, l));
+    });
+}
+
+// embed_rows(idx, coef, rowsize, seed)
+PyObject *py_embed_rows(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
     return guarded([&]() -> PyObject * {
         count_args(n, 4);
-        const Tensor &c = tensor_arg(a[0]);
-        const OptTensor sb = opt_arg(a[1]);
-        const int64_t len = int_arg(a[2]), seed = seed_arg(a[3]);
-        if (!at::GradMode::is_enabled() || !(c.requires_grad() || wants_grad(sb))) return THPVariable_Wrap(VectorFromCoefs::values(c, sb, len, seed));
-        return THPVariable_Wrap(VectorFromCoefs::apply(c, sb, len, seed));
+        const Tensor &idx = tensor_arg(a[0]), &c = tensor_arg(a[1]);
+        const int64_t rowsize = int_arg(a[2]), seed = seed_arg(a[3]);
+        if (!at::GradMode::is_enabled() || !c.requires_grad()) return THPVariable_Wrap(EmbedRows::forward(nullptr, idx, c, rowsize, seed));
+        return THPVariable_Wrap(EmbedRows::apply(idx, c, rowsize, seed));
     });
 }
 
@@ -704,9 +924,9 @@ PyObject *py_set_hooks(PyObject *, PyObject *const *a, Py_ssize_t n)
 
 #define RDB_METHOD(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {RDB_METHOD(takes_projected),   RDB_METHOD(linear_projected), RDB_METHOD(linear_one_call),
-                         RDB_METHOD(vector_from_coefs), RDB_METHOD(set_hooks),        RDB_METHOD(rms_norm),
-                         RDB_METHOD(add_rms_norm),      RDB_METHOD(relu_square),      RDB_METHOD(cross_entropy),
-                         RDB_METHOD(causal_attention),  {nullptr, nullptr, 0, nullptr}};
+                         RDB_METHOD(linear_vector),     RDB_METHOD(embed_rows),       RDB_METHOD(set_hooks),
+                         RDB_METHOD(rms_norm),          RDB_METHOD(add_rms_norm),     RDB_METHOD(relu_square),
+                         RDB_METHOD(cross_entropy),     RDB_METHOD(causal_attention), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_rdb_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
@@ -723,7 +943,10 @@ PyMODINIT_FUNC PyInit__rdb_torch(void)
 {
     name_node<OneCallLinear>("OneCallLinearBackward");
     name_node<ProjectedLinear>("ProjectedLinearBackward");
-    name_node<VectorFromCoefs>("VectorFromCoefsBackward");
+    name_node<VectorLinear>("VectorLinearBackward");
+    name_node<EmbedRows>("EmbedRowsBackward");
+    name_node<CoefValues>("CoefValuesBackward");
+    name_node<CoefGrads>("CoefGradsBackward");
     name_node<RmsNorm>("RmsNormBackward");
     name_node<AddRmsNorm>("AddRmsNormBackward");
     name_node<ReluSquare>("ReluSquareBackward");

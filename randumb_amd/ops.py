@@ -373,15 +373,24 @@ class _ProjectedFunction(torch.autograd.Function):
         return dx, dcoefs, None, None, None, dbias, dsb
 
 
-def _rbias_dense(t) -> Optional[Tensor]:
-    """A layer's pseudorandom bias as a dense tensor with autograd behind it (its coefficients and scale), or None where the
-    tensor is not a contiguous vector-coef one in its coefficients' dtype."""
-    if t.coef_rows or t.dim() != 1 or t.stride(0) != 1 or t.dtype != t._coef.dtype or type(t._coef) not in (Tensor, torch.nn.Parameter):
+def _coef_form(t) -> Optional[tuple]:
+    """``(coefs, scale or None, seed)`` of a contiguous vector-coef tensor in its coefficients' dtype, as the extension module takes
+    a pseudorandom bias or weight (autograd then reaches the coefficients there); None for other pseudorandom tensors."""
+    if t.coef_rows or t.dtype != t._coef.dtype or type(t._coef) not in (Tensor, torch.nn.Parameter) or not t.is_contiguous():
         return None
     c, sb = t._coef, t.scale_bias if t.fused_bias else None
+    if t.fused_bias and sb is None:
+        return None
     if not t.requires_grad:
         c, sb = c.detach(), None if sb is None else sb.detach()
-    return _lib.extension().vector_from_coefs(c, sb, t.shape[0], t.seed)
+    return c, sb, t.seed
+
+
+def _bias_form(bias) -> Optional[tuple]:
+    """The three arguments the extension module takes for a bias; None where it does not take this one."""
+    if bias is None or not hasattr(bias, "get_materialized"):
+        return bias, None, -1
+    return _coef_form(bias) if bias.dim() == 1 else None
 
 
 class _ProjectedLinear:
@@ -390,9 +399,10 @@ class _ProjectedLinear:
 
     @staticmethod
     def apply(x, coefs, in_features, out_features, seed, bias, scale_bias=None):
-        if _tracing() or hip.CHECK_STATE_COEF or hasattr(bias, "get_materialized"):
+        form = None if _tracing() or hip.CHECK_STATE_COEF else _bias_form(bias)
+        if form is None:
             return _ProjectedFunction.apply(x, coefs, in_features, out_features, seed, bias, scale_bias)
-        return _lib.extension().linear_projected(x, coefs, in_features, out_features, seed, bias, scale_bias)
+        return _lib.extension().linear_projected(x, coefs, in_features, out_features, seed, *form, scale_bias)
 
 
 def linear(x: Tensor, coefs: Tensor, in_features: int, out_features: int, stride_o: int, stride_i: int, seed: int,
@@ -402,14 +412,12 @@ def linear(x: Tensor, coefs: Tensor, in_features: int, out_features: int, stride
     ``rten::linear_fwd`` otherwise.  Same arguments as ``rten::linear_fwd``."""
     if x.is_cuda and not _tracing():
         ext = _lib._ext or _lib.extension()
-        if hasattr(bias, "get_materialized"):
-            dense = _rbias_dense(bias)
-            bias = bias if dense is None else dense
         if ext.takes_projected(x, coefs, in_features, out_features, stride_o, stride_i, scale_bias, bias):
             return _ProjectedLinear.apply(x, coefs, in_features, out_features, seed, bias, scale_bias)
-        if hasattr(bias, "get_materialized"):
+        form = _bias_form(bias)
+        if form is None:
             return _OneCallFunction.apply(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias)
-        return ext.linear_one_call(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias)
+        return ext.linear_one_call(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, *form)
     rbias_ok = scale_bias is None or (x.dtype == torch.bfloat16 and scale_bias.numel() == 1 and not _tracing()
                                       and hip.linear_rbias_supported(in_features, out_features, x.dtype))
     if (rbias_ok and coefs.dim() == 2 and coefs.shape[0] == out_features and stride_o == in_features and stride_i == 1
@@ -418,6 +426,26 @@ def linear(x: Tensor, coefs: Tensor, in_features: int, out_features: int, stride
             and hip.linear_projection_preferred(x.shape[0], in_features, out_features, coefs.shape[1], x.dtype)):
         return _ProjectedLinear.apply(x, coefs, in_features, out_features, seed, bias, scale_bias)
     return linear_fwd(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias)
+
+
+def vector_linear(x: Tensor, weight, bias) -> Optional[Tensor]:
+    """``F.linear(x, weight, bias)`` for a vector-coef weight that is formed and multiplied as a dense matrix, without the tensor
+    subclass's dispatch (three operators of torch.library and as many autograd nodes: 480 us of host time for a step whose
+    kernels take 60); None where the request is another one."""
+    if (not x.is_cuda or x.dim() < 2 or type(x) not in (Tensor, torch.nn.Parameter) or x.dtype not in (torch.float32, torch.bfloat16)
+            or x.dtype != weight.dtype or weight.dim() != 2 or x.shape[-1] != weight.shape[1] or _tracing() or torch.is_autocast_enabled()):
+        return None
+    w, b = _coef_form(weight), _bias_form(bias)
+    if w is None or b is None or x.device != w[0].device:
+        return None
+    return (_lib._ext or _lib.extension()).linear_vector(x, w[0], weight.shape[1], weight.shape[0], w[2], w[1], *b)
+
+
+def embed_rows(idx: Tensor, coefs: Tensor, rowsize: int, seed: int) -> Tensor:
+    """``rten::embed_fwd`` with its backward; eagerly on the GPU by the extension module."""
+    if idx.is_cuda and coefs.is_cuda and not _tracing():
+        return (_lib._ext or _lib.extension()).embed_rows(idx, coefs, rowsize, seed)
+    return embed_fwd(idx, coefs, rowsize, seed)
 
 
 # ------------------------------------------------------------------------------------------------ rten_cpp::*

@@ -172,7 +172,8 @@ enum {
 };
 
 enum { RDB_OP_LINEAR_FWD = 0, RDB_OP_LINEAR_BWD_DX = 1, RDB_OP_LINEAR_BWD_DCOEF = 2, RDB_OP_LINEAR_BWD_PROJECTED = 3,
-       RDB_OP_LINEAR_BWD_PROJECTED_TO = 4, RDB_OP_LINEAR_BWD_DX_DSCALE = 5, RDB_OP_LINEAR_RBIAS_BWD = 6 };
+       RDB_OP_LINEAR_BWD_PROJECTED_TO = 4, RDB_OP_LINEAR_BWD_DX_DSCALE = 5, RDB_OP_LINEAR_RBIAS_BWD = 6,
+       RDB_OP_LINEAR_BWD_KEPT = 7 };
 
 /* Device scratch (bytes) that entry point `op` can use for `desc`; 0 when it has no use for any.  A NULL or too small
  * workspace is never an error with RDB_ALGO_AUTO: the library then runs a kernel that needs none. */
@@ -339,6 +340,20 @@ int rdb_linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *d
 int rdb_linear_bwd_projected_to(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, const void *dy, int64_t lddy,
                                 const void *state, const void *coef, const rdb_linear_desc *desc, void *workspace,
                                 int64_t workspace_bytes, void *stream);
+
+/* The projected form's counterpart for layers without a projection state (bf16 with sizes that are not multiples of 8, fp32
+ * in the few-token regime; rdb_linear_kept_bytes says how much, 0: none, use the calls above): the forward pass leaves
+ * z = x . N^T (fp32, [tokens x k] row-major) in `kept`, 16-byte aligned, and the backward pass starts from it.  scale_bias as
+ * in rdb_linear_fwd.  rdb_linear_bwd_kept: dx, dcoef (dcoef_dtype RDB_F32 or RDB_BF16) and d_scale_bias (fp32) are
+ * overwritten, NULL where not wanted; x is read for d_scale_bias only; a workspace of
+ * rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_KEPT, desc) bytes.  Sums in a fixed order. */
+int64_t rdb_linear_kept_bytes(const rdb_linear_desc *desc);
+int rdb_linear_fwd_kept(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef,
+                        const void *scale_bias, const void *bias, const rdb_linear_desc *desc, void *stream);
+int rdb_linear_bwd_kept(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy,
+                        int64_t lddy, const void *x, int64_t ldx, const void *kept, const void *coef,
+                        const void *scale_bias, const rdb_linear_desc *desc, void *workspace, int64_t workspace_bytes,
+                        void *stream);
 
 /* For tools that time the two kernel launches of rdb_linear_bwd_projected one by one (no counterpart in the reference):
  * part 1 enqueues only the first launch (dy.C into the workspace and the partial sums of dcoef), part 2 only the second

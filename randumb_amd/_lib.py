@@ -17,6 +17,7 @@ RDB_ALGO_AUTO, RDB_ALGO_TILE, RDB_ALGO_STRIP, RDB_ALGO_FACTORED = 0, 1, 2, 3
 RDB_OP_LINEAR_FWD, RDB_OP_LINEAR_BWD_DX, RDB_OP_LINEAR_BWD_DCOEF, RDB_OP_LINEAR_BWD_PROJECTED, RDB_OP_LINEAR_BWD_PROJECTED_TO = 0, 1, 2, 3, 4
 RDB_OP_LINEAR_BWD_DX_DSCALE = 5
 RDB_OP_LINEAR_RBIAS_BWD = 6
+RDB_OP_LINEAR_BWD_KEPT = 7
 
 # every exported entry point, in header order; tests check the list against the built library
 EXPORTS = [
@@ -56,6 +57,9 @@ EXPORTS = [
     "rdb_linear_bwd_projected",
     "rdb_linear_bwd_projected_to",
     "rdb_linear_bwd_projected_part",
+    "rdb_linear_kept_bytes",
+    "rdb_linear_fwd_kept",
+    "rdb_linear_bwd_kept",
     "rdb_set_big_tiles",
     "rdb_set_f32_split",
     "rdb_set_one_launch",
@@ -189,6 +193,12 @@ def load() -> ctypes.CDLL:
     L.rdb_linear_bwd_projected.argtypes = [vp, i64, vp, vp, i64, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_bwd_projected_to.argtypes = [vp, i64, vp, ci, vp, i64, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_bwd_projected_part.argtypes = [ci, vp, i64, vp, vp, i64, vp, vp, dp, vp, i64, vp]
+    L.rdb_linear_kept_bytes.argtypes = [dp]
+    L.rdb_linear_kept_bytes.restype = i64
+    L.rdb_linear_fwd_kept.argtypes = [vp, i64, vp, vp, i64, vp, vp, vp, dp, vp]
+    L.rdb_linear_fwd_kept.restype = ci
+    L.rdb_linear_bwd_kept.argtypes = [vp, i64, vp, ci, vp, vp, i64, vp, i64, vp, vp, vp, dp, vp, i64, vp]
+    L.rdb_linear_bwd_kept.restype = ci
     L.rdb_set_big_tiles.argtypes = [ci]
     L.rdb_set_big_tiles.restype = ci
     L.rdb_set_f32_split.argtypes = [ci]

@@ -230,6 +230,105 @@ int linear_dcoef_f32(float *dcoef, float *d_scale_bias, const void *dy, int64_t 
     return check_launch("f32_sum_scalars_kernel");
 }
 
+// ----------------------------------------------------------------------------------------------- z kept from forward to backward
+// For the layers that have no projection state of their own (bf16 with sizes that are not multiples of 8, fp32 in the few-token
+// regime): the forward pass leaves z = x . N^T, [tokens x k] in fp32, and the backward pass takes it from there instead of
+// projecting x again.  Only while that is at most twice the size of x, which the caller keeps too.  Few tokens (in fp32 below 32,
+// in bf16 up to 96) stay with the kernels of rdb_smallk.hip.  4097 tokens x 1001 -> 999, k = 100 in bf16, forward and backward:
+// 122 -> 98 us; 128 tokens x 784 -> 256, k = 64 in fp32: 22.7 + 11.1 + 27.8 us of few-token kernels -> 17 + 6.
+int64_t linear_kept_f32_bytes(const rdb_linear_desc *d)
+{
+    if (!fg_ok(d) || d->algo != RDB_ALGO_AUTO || d->tokens * std::max(d->in_f, d->out_f) >= (1ll << 28) || d->sO != d->in_f || d->sI != 1) return 0;
+    const bool b16 = d->act_dtype == RDB_BF16;
+    if (b16 ? (d->tokens <= 96 || !(d->in_f % 8 || d->out_f % 8 || d->k % 8) || d->k > d->in_f) : (d->tokens < 32 || d->k > 2 * d->in_f)) return 0;
+    return up256(d->tokens * d->k * 4);
+}
+
+static int fg_rbias(FgProduct q, const void *scale, const rdb_linear_desc *d, int num_cus, hipStream_t s, const char *name)
+{
+    q.a_es = fg_es(d->act_dtype);
+    q.out_bf16 = d->act_dtype == RDB_BF16;
+    q.scale = static_cast<const float *>(scale);
+    q.scale_bf16 = d->coef_dtype == RDB_BF16;
+    return fg_launch<FG_KCONT, FG_NOISE_1D>(q, num_cus, s, name);
+}
+
+int linear_fwd_kept_f32(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
+                        const rdb_linear_desc *d, int num_cus, hipStream_t s)
+{
+    if (!linear_kept_f32_bytes(d) || !fg_aligned16(kept) || d->tokens * ldx >= (1ll << 29) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
+    float *z = static_cast<float *>(kept);
+    // the partial matrices of the projection's ranges lie in y's memory, which is written last
+    const bool room = ldy == d->out_f && fg_aligned16(y);
+    const int max_ranges = room ? (int)std::min<int64_t>(32, d->tokens * d->out_f * fg_es(d->act_dtype) / up256(d->tokens * d->k * 4)) : 1;
+    if (int rc = fg_project(z, (const float *)x, ldx, d, num_cus, s, room ? (float *)y : z, max_ranges)) return rc;
+    FgProduct q = {z, d->k, d->tokens * d->k, (const float *)coef, d->k, d->out_f * d->k, (float *)y, ldy, (const float *)bias, d->tokens, d->out_f, d->k,
+                   0, 0, 0, 0, d->seed};
+    q.b_es = fg_es(d->coef_dtype);
+    q.out_bf16 = d->act_dtype == RDB_BF16;
+    if (int rc = fg_launch<FG_KCONT, FG_KCONT>(q, num_cus, s, "f32_gemm_kernel (y = z . C^T)")) return rc;
+    if (!scale_bias) return RDB_OK;
+    FgProduct qr = {(const float *)x, ldx, (d->tokens - 1) * ldx + d->in_f, nullptr, 0, 0, (float *)y, ldy, nullptr, d->tokens, d->out_f, d->in_f,
+                    0, 0, 0, 0, d->seed, (uint32_t)d->in_f, 1u};
+    return fg_rbias(qr, scale_bias, d, num_cus, s, "f32_gemm_kernel (y += s x . R^T)");
+}
+
+// t = dy . C and its partial matrices, those of dC = dy^T . z, and one value per tile of dy . R (at most 64 x 128 of [tokens x in_f] or
+// [tokens x out_f])
+int64_t linear_bwd_kept_f32_workspace(const rdb_linear_desc *d, int num_cus)
+{
+    if (!linear_kept_f32_bytes(d)) return 0;
+    const int r = dc_room(d, num_cus);
+    return linear_f32_workspace(RDB_OP_LINEAR_BWD_DX, d, num_cus) + (r > 1 ? (int64_t)r * up256(d->out_f * d->k * 4) : 0) +
+           up256(cdiv(d->tokens, 64) * cdiv(std::max(d->in_f, d->out_f), FG_BN) * 4);
+}
+
+// dx, dcoef (fp32 or bf16) and d_scale_bias: each NULL where it is not wanted.  With dx wanted, the gradient of the scale, <dy . R, x>,
+// comes out of the random-bias product that dx needs anyway.
+int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x, int64_t ldx,
+                        const void *kept, const void *coef, const void *scale_bias, const rdb_linear_desc *d, int num_cus, void *workspace,
+                        int64_t workspace_bytes, hipStream_t s)
+{
+    if (!linear_kept_f32_bytes(d) || !fg_aligned16(kept) || !workspace || !fg_aligned16(workspace) ||
+        workspace_bytes < linear_bwd_kept_f32_workspace(d, num_cus) || d->tokens * lddy >= (1ll << 29) || (dx && d->tokens * lddx >= (1ll << 29)) ||
+        (d_scale_bias && d->tokens * ldx >= (1ll << 29)))
+        return RDB_E_UNSUPPORTED;
+    char *const dc_part = static_cast<char *>(workspace) + linear_f32_workspace(RDB_OP_LINEAR_BWD_DX, d, num_cus);
+    const int r = dc_room(d, num_cus);
+    float *const dots = reinterpret_cast<float *>(dc_part + (r > 1 ? (int64_t)r * up256(d->out_f * d->k * 4) : 0));
+    if (dx) {
+        if (int rc = linear_dx_f32(dx, lddx, dy, lddy, coef, nullptr, d, num_cus, workspace, workspace_bytes, s)) return rc;
+    }
+    if (dcoef) {
+        FgProduct q = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, static_cast<const float *>(kept), d->k, d->tokens * d->k, (float *)dcoef, d->k,
+                       nullptr, d->out_f, d->k, d->tokens, 0, 0, 0, 0, d->seed};
+        q.a_es = fg_es(d->act_dtype);
+        q.out_bf16 = dcoef_dtype == RDB_BF16;
+        if (int rc = fg_launch_ranges<FG_MCONT, FG_MCONT>(q, r, reinterpret_cast<float *>(dc_part), up256(d->out_f * d->k * 4) / 4, num_cus, s,
+                                                          "f32_gemm_kernel (dC = dy^T . z)"))
+            return rc;
+    }
+    if (!scale_bias || (!dx && !d_scale_bias)) return RDB_OK;
+    FgProduct q;
+    if (dx) {   // dx += s * dy . R, and <dy . R, x> on the way
+        q = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, nullptr, 0, 0, (float *)dx, lddx, nullptr, d->tokens, d->in_f, d->out_f,
+             0, 0, 0, 0, d->seed, 1u, (uint32_t)d->in_f};
+        if (d_scale_bias) q.dotm = (const float *)x, q.lddot = ldx;
+    } else {    // <x . R^T, dy>
+        q = {(const float *)x, ldx, (d->tokens - 1) * ldx + d->in_f, nullptr, 0, 0, nullptr, 0, nullptr, d->tokens, d->out_f, d->in_f,
+             0, 0, 0, 0, d->seed, (uint32_t)d->in_f, 1u};
+        q.dotm = (const float *)dy, q.lddot = lddy;
+    }
+    const FgPlan pl = fg_plan(q.M, q.N, q.K, num_cus, 1, true);
+    q.bm = pl.bm;
+    q.groups = pl.groups;
+    q.dot_part = d_scale_bias ? dots : nullptr;
+    if (int rc = fg_rbias(q, dx ? scale_bias : nullptr, d, num_cus, s, "f32_gemm_kernel (dx += s dy . R)")) return rc;
+    if (!d_scale_bias) return RDB_OK;
+    f32_sum_scalars_kernel<<<1, 256, 0, s>>>(d_scale_bias, dots, (int)(cdiv(q.M, q.bm) * cdiv(q.N, FG_BN)));
+    return check_launch("f32_sum_scalars_kernel");
+}
+
 // ----------------------------------------------------------------------------------------------- dW = dy^T . x on its own
 // For the vector-coef coefficient gradient: every element of dW meets k hashed values, so that gradient is bound by the hash
 // whatever is fused into it, and a kernel that forms dW tile by tile per block of tokens repeats the k hashes per element for

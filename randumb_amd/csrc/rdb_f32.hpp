@@ -25,7 +25,7 @@ enum FgSource {
 enum FgEpilogue {
     FG_STORE = 0,       // out = acc
     FG_STORE_BIAS = 1,  // out = acc + bias[column]
-    FG_ADD_SCALED = 2,  // out += scale[0] * acc
+    FG_ADD_SCALED = 2,  // out += scale[0] * acc; with dotm also the sums of FG_DOT
     FG_DOT = 3,         // dot_part[block] = sum over the tile of acc * dotm (nothing is stored to out)
     FG_STORE_RBIAS = 4  // out = acc + scale[0] * noise1d(row * nsR + column * nsK): materialising W = C . N + s . R
 };
@@ -47,9 +47,9 @@ struct FgParams {
     int scale_bf16;             // scale is bf16 (the coefficients' dtype)
     uint32_t nsR, nsK;          // FG_NOISE_1D: index steps per row and per contraction value
     const float *scale;         // FG_ADD_SCALED: one device value
-    const float *dotm;          // FG_DOT: [M x N] matrix, leading dimension lddot
+    const float *dotm;          // FG_DOT, FG_ADD_SCALED (or NULL): [M x N] matrix, leading dimension lddot
     int64_t lddot;
-    float *dot_part;            // FG_DOT: one value per block, in block order (x fastest, then y)
+    float *dot_part;            // with dotm: one value per block, in block order (x fastest, then y)
 };
 
 // fp32 products on the bf16 matrix cores.  v = h + m + l exactly, each part a bf16 (the top 8 bits of what is left: truncation,
@@ -484,10 +484,11 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
                 const int m = m0 + wm * (BM / 2) + mi * 32 + 8 * (j >> 2) + 4 * g + (j & 3);
                 if (m >= p.M) continue;
                 const float a = acc[mi][ni][j];
-                if (EPI == FG_DOT) {
+                if (EPI == FG_DOT || (EPI == FG_ADD_SCALED && p.dotm)) {
                     const int64_t e = (int64_t)m * p.lddot + n;
                     dot = fmaf(a, o16 ? bf16_to_f32(reinterpret_cast<const bf16_t *>(p.dotm)[e]) : p.dotm[e], dot);
-                } else {
+                }
+                if (EPI != FG_DOT) {
                     const int64_t e = (int64_t)m * p.ldo + n;
                     if (EPI == FG_STORE_RBIAS) out[e] = fmaf(scale, noise1d((uint32_t)m * p.nsR + (uint32_t)n * p.nsK, p.seed), a);
                     else if (o16) out16[e] = f32_to_bf16(EPI == FG_ADD_SCALED ? fmaf(scale, a, bf16_to_f32(out16[e])) : a + bv);
@@ -496,14 +497,19 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
                 }
             }
     }
-    if (EPI == FG_DOT) {
+    if (EPI == FG_DOT || (EPI == FG_ADD_SCALED && p.dotm)) {
         // lanes, then waves, in a fixed order
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) dot += __shfl_xor(dot, o);
         __syncthreads();   // the stage buffers are free
-        if (lane == 0) lds[wave] = dot;
+        if (lane == 0) lds_all[group * 4 + wave] = dot;
         __syncthreads();
-        if (t == 0) p.dot_part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = (lds[0] + lds[1]) + (lds[2] + lds[3]);
+        if (threadIdx.x == 0) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4 * G; ++i) sum += lds_all[i];
+            p.dot_part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = sum;
+        }
     }
 }
 
@@ -590,7 +596,7 @@ struct FgProduct {
     // the random-bias products (FG_NOISE_1D on the B side): index steps, and what the epilogue does
     uint32_t nsR, nsK;
     const float *scale;     // out += scale[0] * product
-    const float *dotm;      // or: dot_part[block] = <product tile, dotm tile>
+    const float *dotm;      // and / or: dot_part[block] = <product tile, dotm tile>
     int64_t lddot;
     float *dot_part;
     // bytes per element of the A and B matrices (2: bf16), and whether out / bias / dotm and scale are bf16
@@ -617,18 +623,17 @@ struct FgProduct {
         else if (vec) f32_gemm_kernel<BM_, 1, ASRC, BSRC, EPI_, true><<<grid, FG_THREADS, 0, s>>>(p);               \
         else f32_gemm_kernel<BM_, 1, ASRC, BSRC, EPI_, false><<<grid, FG_THREADS, 0, s>>>(p);                       \
     } while (0)
-// What is built for a pair of sources: several groups per block (four groups' buffers do not fit in LDS where a side is read
+// What is built for a pair of sources: four groups per block (their buffers do not fit in LDS where a side is read
 // across its rows: its planes are padded), and the epilogues that add a bias and a random-bias share.
 template <int ASRC, int BSRC> struct FgGroups {
-    static constexpr bool any = BSRC != FG_NOISE_1D, four = any && ASRC != FG_MCONT && BSRC != FG_MCONT;
+    static constexpr bool four = ASRC != FG_MCONT && BSRC != FG_MCONT;
     static constexpr bool biased = ASRC == FG_KCONT && BSRC == FG_KCONT, scaled = ASRC == FG_NOISE_I || BSRC == FG_NOISE_I;
 };
 template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_t s, const char *name)
 {
     typedef FgGroups<ASRC, BSRC> Groups;
     if (!q.bm) {
-        const bool plain = Groups::any && !q.scale;
-        const FgPlan pl = plain ? fg_plan(q.M, q.N, q.K, num_cus, 1, Groups::four) : fg_room(q.M, q.N, q.K, num_cus, q.K, 1);
+        const FgPlan pl = !(Groups::scaled && q.scale) ? fg_plan(q.M, q.N, q.K, num_cus, 1, Groups::four) : fg_room(q.M, q.N, q.K, num_cus, q.K, 1);
         q.bm = pl.bm;
         q.groups = pl.groups;
     }
@@ -670,28 +675,23 @@ template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_
     const bool any16 = q.a_es == 2 || ((BSRC == FG_KCONT || BSRC == FG_MCONT) && q.b_es == 2);   // the A side is always a matrix
     if (cdiv(q.N, FG_BN) > 65535) return RDB_E_UNSUPPORTED;   // the grid's y
     const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)splits);
-    if constexpr (BSRC == FG_NOISE_1D) {   // the random-bias products: added on top of an output, or reduced against a matrix
-        if (q.bm == 128) {
-            if (q.dotm) FG_LAUNCH(128, FG_DOT);
-            else FG_LAUNCH(128, FG_ADD_SCALED);
-        } else {
-            if (q.dotm) FG_LAUNCH(64, FG_DOT);
-            else FG_LAUNCH(64, FG_ADD_SCALED);
-        }
+    auto run = [&](auto epi_) {
+        constexpr int EPI = decltype(epi_)::value;
+        if (q.bm == 128 && q.groups == 2) FG_LAUNCH_GROUPS(128, 2, EPI);
+        else if (q.bm == 128) FG_LAUNCH(128, EPI);
+        else if (q.groups == 1) FG_LAUNCH(64, EPI);
+        else if (q.groups == 2) FG_LAUNCH_GROUPS(64, 2, EPI);
+        else if constexpr (Groups::four) FG_LAUNCH_GROUPS(64, 4, EPI);
+    };
+    if constexpr (BSRC == FG_NOISE_1D) {   // the random-bias products: added on top of an output, and / or reduced against a matrix
+        if (q.scale) run(std::integral_constant<int, FG_ADD_SCALED>{});
+        else run(std::integral_constant<int, FG_DOT>{});
     } else if (Groups::scaled && q.scale) {   // materialising W with its random-bias share
         if constexpr (Groups::scaled) {
             if (q.bm == 128) FG_LAUNCH(128, FG_STORE_RBIAS);
             else FG_LAUNCH(64, FG_STORE_RBIAS);
         }
     } else {
-        auto run = [&](auto epi_) {
-            constexpr int EPI = decltype(epi_)::value;
-            if (q.bm == 128 && q.groups == 2) FG_LAUNCH_GROUPS(128, 2, EPI);
-            else if (q.bm == 128) FG_LAUNCH(128, EPI);
-            else if (q.groups == 1) FG_LAUNCH(64, EPI);
-            else if (q.groups == 2) FG_LAUNCH_GROUPS(64, 2, EPI);
-            else if constexpr (Groups::four) FG_LAUNCH_GROUPS(64, 4, EPI);
-        };
         if constexpr (Groups::biased) {
             if (q.bias) run(std::integral_constant<int, FG_STORE_BIAS>{});
             else run(std::integral_constant<int, FG_STORE>{});

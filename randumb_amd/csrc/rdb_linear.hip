@@ -416,10 +416,14 @@ static int64_t vec_dcoef_workspace(const rdb_linear_desc *d)
 }
 
 static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d);
+namespace rdb {
+int64_t linear_bwd_kept_f32_workspace(const rdb_linear_desc *d, int num_cus);   // rdb_f32.hip
+}
 
 extern "C" int64_t rdb_linear_workspace_bytes(int op, const rdb_linear_desc *d)
 {
     if (!d) return 0;
+    if (op == RDB_OP_LINEAR_BWD_KEPT) return rdb_linear_kept_bytes(d) ? linear_bwd_kept_f32_workspace(d, num_compute_units()) : 0;
     int64_t need = linear_workspace_bytes_main(op, d);
     if (d->algo == RDB_ALGO_AUTO && d->act_dtype == RDB_BF16 && d->coef_rows != 0 &&
         (op == RDB_OP_LINEAR_FWD || op == RDB_OP_LINEAR_BWD_DX || op == RDB_OP_LINEAR_BWD_DCOEF)) {
@@ -1191,6 +1195,52 @@ extern "C" int rdb_linear_bwd_projected_to(void *dx, int64_t lddx, void *dcoef, 
                                            const void *coef, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
 {
     return bwd_projected_entry("rdb_linear_bwd_projected_to", dx, lddx, dcoef, dcoef_dtype, dy, lddy, z, coef, d, workspace, workspace_bytes, stream);
+}
+
+// ----------------------------------------------------------------------------------------------- z kept from forward to backward
+namespace rdb {   // rdb_f32.hip
+int64_t linear_kept_f32_bytes(const rdb_linear_desc *d);
+int linear_fwd_kept_f32(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
+                        const rdb_linear_desc *d, int num_cus, hipStream_t s);
+int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x, int64_t ldx,
+                        const void *kept, const void *coef, const void *scale_bias, const rdb_linear_desc *d, int num_cus, void *workspace,
+                        int64_t workspace_bytes, hipStream_t s);
+}
+
+extern "C" int64_t rdb_linear_kept_bytes(const rdb_linear_desc *d)
+{
+    if (check_desc("rdb_linear_kept_bytes", d) || rdb_linear_projection_preferred(d)) return 0;
+    return linear_kept_f32_bytes(d);
+}
+
+extern "C" int rdb_linear_fwd_kept(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
+                                   const rdb_linear_desc *d, void *stream)
+{
+    if (int rc = check_desc("rdb_linear_fwd_kept", d)) return rc;
+    if (!rdb_linear_kept_bytes(d)) return set_error(RDB_E_UNSUPPORTED, "rdb_linear_fwd_kept: a layer of which nothing is kept (rdb_linear_kept_bytes)");
+    if (!y || !kept || !x || !coef) return set_error(RDB_E_NULL, "rdb_linear_fwd_kept: y, kept, x or coef is NULL");
+    if (ldx < d->in_f || ldy < d->out_f) return set_error(RDB_E_SHAPE, "rdb_linear_fwd_kept: leading dimension smaller than the row");
+    const int rc = linear_fwd_kept_f32(y, ldy, kept, x, ldx, coef, scale_bias, bias, d, num_compute_units(), (hipStream_t)stream);
+    return rc == RDB_E_UNSUPPORTED ? set_error(rc, "rdb_linear_fwd_kept: kept must be 16-byte aligned and tokens * ldx, tokens * ldy below 2^29") : rc;
+}
+
+extern "C" int rdb_linear_bwd_kept(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x,
+                                   int64_t ldx, const void *kept, const void *coef, const void *scale_bias, const rdb_linear_desc *d, void *workspace,
+                                   int64_t workspace_bytes, void *stream)
+{
+    if (int rc = check_desc("rdb_linear_bwd_kept", d)) return rc;
+    if (!rdb_linear_kept_bytes(d)) return set_error(RDB_E_UNSUPPORTED, "rdb_linear_bwd_kept: a layer of which nothing is kept (rdb_linear_kept_bytes)");
+    if (!dy || (dx && !coef) || (dcoef && !kept) || (d_scale_bias && (!x || !scale_bias)))
+        return set_error(RDB_E_NULL, "rdb_linear_bwd_kept: dy, x, kept, coef or scale_bias is NULL");
+    if (lddy < d->out_f || (dx && lddx < d->in_f) || (d_scale_bias && ldx < d->in_f))
+        return set_error(RDB_E_SHAPE, "rdb_linear_bwd_kept: leading dimension smaller than the row");
+    if (dcoef_dtype != RDB_F32 && dcoef_dtype != RDB_BF16) return set_error(RDB_E_DTYPE, "rdb_linear_bwd_kept: unknown dcoef dtype %d", dcoef_dtype);
+    const int rc = linear_bwd_kept_f32(dx, lddx, dcoef, dcoef_dtype, d_scale_bias, dy, lddy, x, ldx, kept, coef, scale_bias, d, num_compute_units(), workspace,
+                                       workspace_bytes, (hipStream_t)stream);
+    if (rc == RDB_E_UNSUPPORTED)
+        return set_error(rc, "rdb_linear_bwd_kept: needs a 16-byte aligned workspace of rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_KEPT) bytes and tokens "
+                             "times each leading dimension below 2^29");
+    return rc;
 }
 
 // rdb_factored.hip, rdb_smallk.hip

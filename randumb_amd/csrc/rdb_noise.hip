@@ -2,6 +2,7 @@
 // These are the HBM-facing ops of the pseudorandom tensor (the fused linear kernels live in rdb_linear.hip).
 #include "rdb_common.hpp"
 #include <algorithm>
+#include <type_traits>
 
 namespace rdb {
 
@@ -60,31 +61,37 @@ struct MatVecParams {
     uint32_t seed;
 };
 
-template <bool GATHER> __global__ __launch_bounds__(NT) void materialize_vec_kernel(MatVecParams p)
+// LANES > 1: that many neighbouring lanes share an element, lane l its terms l, l + LANES, .. (then added up across the lanes, nearest
+// first): with few elements the chip is not full, and the chain's length is what a launch takes (3072 elements, k = 256: 16.5 ->
+// 4 us).
+template <bool GATHER, int LANES> __global__ __launch_bounds__(NT) void materialize_vec_kernel(MatVecParams p)
 {
     __shared__ float cs[COEF_CHUNK];
-    const int64_t n = (int64_t)blockIdx.x * NT + threadIdx.x;
+    const int64_t n = ((int64_t)blockIdx.x * NT + threadIdx.x) / LANES;
+    const int part = threadIdx.x % LANES;
     const bool live = n < p.Nw;
     uint32_t a = (uint32_t)n;
     if (live && (GATHER || !p.contiguous)) {
         const int64_t r = p.narrow ? (int64_t)((uint32_t)n / (uint32_t)p.Q) : n / p.Q, q = n - r * p.Q;
         a = GATHER ? (uint32_t)(p.idx[r] * p.Q + q) : (uint32_t)(q * p.sQ + r * p.sP);
     }
-    uint32_t first = a * PN1 + p.seed;  // first-round value for m = 0; +N1 per step of m
+    uint32_t first = a * PN1 + p.seed + (uint32_t)part * SQ5_N1;  // first-round value for m = part; +N1 per step of m
     float acc = 0.0f;
-    for (int64_t m0 = 0; m0 < p.k; m0 += COEF_CHUNK) {
+    for (int64_t m0 = 0; m0 < p.k; m0 += COEF_CHUNK) {   // a multiple of LANES
         const int cnt = (int)((p.k - m0) < COEF_CHUNK ? (p.k - m0) : COEF_CHUNK);
         __syncthreads();
         for (int j = threadIdx.x; j < cnt; j += NT) cs[j] = load_as_f32(p.coef, p.coef_dtype, m0 + j);
         __syncthreads();
         if (live) {
-            for (int j = 0; j < cnt; ++j) {
+            for (int j = part; j < cnt; j += LANES) {
                 acc = fmaf(sq5_unit(sq5_tail_apart(first)), cs[j], acc);
-                first += SQ5_N1;
+                first += LANES * SQ5_N1;
             }
         }
     }
-    if (live) {
+#pragma unroll
+    for (int w = 1; w < LANES; w *= 2) acc += __shfl_xor(acc, w);
+    if (live && part == 0) {
         if (p.scale_bias) acc += load_as_f32(p.scale_bias, p.coef_dtype, 0) * noise1d(a, p.seed);
         p.out[n] = acc;
     }
@@ -453,8 +460,17 @@ static int launch_materialize_vec(float *out, const void *coef, int coef_dtype, 
                                   const void *scale_bias, const int64_t *idx, hipStream_t s)
 {
     const MatVecParams p = {out, coef, scale_bias, idx, k, Nw, Q, sP, sQ, coef_dtype, Nw < (1ll << 32) && Q < (1ll << 32), sQ == 1 && (sP == Q || Nw == Q), seed};
-    if (idx) materialize_vec_kernel<true><<<(unsigned)cdiv(Nw, NT), NT, 0, s>>>(p);
-    else materialize_vec_kernel<false><<<(unsigned)cdiv(Nw, NT), NT, 0, s>>>(p);
+    // lanes per element: as many as fill the chip's 8192 wave slots, of 1, 4, 16
+    const int lanes = k < 8 ? 1 : Nw <= (1 << 15) ? 16 : Nw <= (1 << 17) ? 4 : 1;
+    const unsigned blocks = (unsigned)cdiv(Nw * lanes, NT);
+    auto launch = [&](auto lanes_) {
+        constexpr int L = decltype(lanes_)::value;
+        if (idx) materialize_vec_kernel<true, L><<<blocks, NT, 0, s>>>(p);
+        else materialize_vec_kernel<false, L><<<blocks, NT, 0, s>>>(p);
+    };
+    if (lanes == 16) launch(std::integral_constant<int, 16>{});
+    else if (lanes == 4) launch(std::integral_constant<int, 4>{});
+    else launch(std::integral_constant<int, 1>{});
     return check_launch("materialize_vec_kernel");
 }
 
@@ -751,8 +767,14 @@ __global__ __launch_bounds__(NT) void bias_grad_kernel(float *__restrict__ dcoef
     const bool scale = !dcoef || m0 >= k;
     float acc[BIAS_M] = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int64_t o = threadIdx.x; o < n; o += NT) {
-        float g = part[o];
-        for (int c = 1; c < chunks; ++c) g += part[(int64_t)c * n + o];
+        float g = 0.0f;
+        for (int c0 = 0; c0 < chunks; c0 += 8) {   // eight loads in flight
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = part[(int64_t)(c0 + i < chunks ? c0 + i : chunks - 1) * n + o];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) g += c0 + i < chunks ? v[i] : 0.0f;
+        }
         if (scale) {
             acc[0] = fmaf(g, noise1d((uint32_t)o, seed), acc[0]);
         } else {

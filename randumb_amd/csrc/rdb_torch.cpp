@@ -253,30 +253,62 @@ std::pair<Tensor, Tensor> linear_bwd_dcoef(const Tensor &dy0, const Tensor &x0, 
 rdb_linear_desc rbias_desc(const Tensor &rows, const Layer &l) { return desc(rows.size(0), l, 8, l.out_f, at::kBFloat16, at::kBFloat16); }
 
 // ----------------------------------------------------------------------------------------------- one-call form
-// y = x.W^T (+ bias) with x saved; the three products of the layer as three calls.
+// y = x.W^T (+ bias) with x saved; the three products of the layer as three calls, or, for the layers of which the library keeps
+// z = x.N^T (rdb_linear_kept_bytes), that saved and one call each way.
 class OneCallLinear : public Function<OneCallLinear> {
   public:
-    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &coefs, const OptTensor &scale_bias, const OptTensor &bias,
+    static Tensor forward(AutogradContext *ctx, const Tensor &x0, const Tensor &coefs, const OptTensor &scale_bias, const OptTensor &bias,
                           const OptTensor &bias_scale, int64_t bias_seed, const Layer &l)
     {
         const Bias b{bias, bias_scale, bias_seed};
-        ctx->save_for_backward({x, coefs, scale_bias.value_or(Tensor())});
         ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, l.sO, l.sI, (int64_t)l.seed, scale_bias ? 1 : 0};
         ctx->saved_data["bias"] = b.meta();
-        return linear_fwd(x, coefs, l, scale_bias, b);
+        const Tensor x = act(x0);
+        const bool same = x.scalar_type() == coefs.scalar_type() && readable(coefs.scalar_type()) && (!scale_bias || scale_bias->numel() == 1);
+        const rdb_linear_desc d = desc(x, l, coefs);
+        const int64_t keep = same && coefs.dim() == 2 && coefs.size(0) == l.out_f ? rdb_linear_kept_bytes(&d) : 0;
+        if (!keep) {
+            ctx->save_for_backward({x0, coefs, scale_bias.value_or(Tensor()), Tensor()});
+            return linear_fwd(x0, coefs, l, scale_bias, b);
+        }
+        const c10::OptionalDeviceGuard guard(x.device());
+        const Tensor c = coefs.contiguous(), sb = scale_bias ? scale_bias->to(c.scalar_type()) : Tensor(), bv = b.values(l.out_f, x.scalar_type());
+        Tensor y = at::empty({x.size(0), l.out_f}, x.options()), kept = bytes(keep, x);
+        check(rdb_linear_fwd_kept(y.data_ptr(), l.out_f, kept.data_ptr(), x.data_ptr(), x.stride(0), c.data_ptr(), ptr(sb), ptr(bv), &d, stream_of(x)),
+              "rdb_linear_fwd_kept");
+        ctx->save_for_backward({scale_bias ? x0 : Tensor(), coefs, scale_bias.value_or(Tensor()), kept});
+        return y;
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &x = saved[0], &coefs = saved[1], &sb = saved[2];
+        const Tensor &x = saved[0], &coefs = saved[1], &sb = saved[2], &kept = saved[3];
         const auto m = ctx->saved_data["layer"].toIntVector();
         const Layer l{m[0], m[1], m[2], m[3], (uint32_t)m[4]};
         const bool has_sb = m[5] != 0;
         const at::AutoGradMode no_grad(false);
         const bool want_dx = ctx->needs_input_grad(0), want_dc = ctx->needs_input_grad(1);
         bool want_sb = has_sb && ctx->needs_input_grad(2);
-        const Tensor dy = grads[0].contiguous();
+        const Tensor dy = kept.defined() ? act(grads[0]) : grads[0].contiguous();
         Tensor dx, dc, dsb;
+        if (kept.defined()) {
+            if (want_dx || want_dc || want_sb) {
+                const c10::OptionalDeviceGuard guard(dy.device());
+                const Tensor c = coefs.contiguous(), xs = want_sb ? act(x) : Tensor(), s = has_sb ? sb.to(c.scalar_type()) : Tensor();
+                const rdb_linear_desc d = desc(dy, l, c);
+                if (want_dx) dx = at::empty({dy.size(0), l.in_f}, dy.options());
+                if (want_dc) dc = at::empty({c.size(0), c.size(1)}, c.options());
+                if (want_sb) dsb = at::empty({1}, dy.options().dtype(at::kFloat));
+                const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_KEPT, &d);
+                const Tensor ws = bytes(need, dy);
+                check(rdb_linear_bwd_kept(ptr(dx), l.in_f, ptr(dc), code(c.scalar_type()), want_sb ? dsb.data_ptr<float>() : nullptr, dy.data_ptr(), dy.stride(0),
+                                          ptr(xs), want_sb ? xs.stride(0) : l.in_f, kept.data_ptr(), c.data_ptr(), ptr(s), &d, ptr(ws), need, stream_of(dy)),
+                      "rdb_linear_bwd_kept");
+                if (want_sb) dsb = dsb.to(sb.scalar_type());
+            }
+            const auto db = bias_grads(ctx, dy, ctx->saved_data["bias"].toIntVector(), has_sb ? 3 : 2);
+            return {dx, dc, dsb, db.first, db.second, Tensor(), Tensor()};
+        }
         if (want_dx && want_sb && l.sO == l.in_f && l.sI == 1) {
             // the random-bias product dy.R that dx needs anyway also gives the gradient of the bias's scale (reduced against x
             // in the same pass), so the coefficient gradient below comes from the factored kernels and dW is never formed

@@ -1,0 +1,61 @@
+"""Layers whose forward pass keeps z = x . N^T for the backward pass (bf16 with odd sizes, fp32 in the few-token regime): against
+float64, at both ends of the range, with the fused random bias and with gradients that are not wanted."""
+import ctypes
+
+import pytest
+import torch
+
+from randumb_amd import _lib, hip, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    return float((a.double().cpu() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("T,in_f,out_f,k,dtype", [(32, 784, 256, 64, torch.float32), (128, 256, 10, 64, torch.float32), (500, 999, 77, 33, torch.float32),
+                                                  (97, 1001, 130, 100, torch.bfloat16), (1200, 260, 515, 71, torch.bfloat16)])
+@pytest.mark.parametrize("rbias", [False, True])
+def test_against_float64(T, in_f, out_f, k, dtype, rbias):
+    g = torch.Generator().manual_seed(T)
+    x, dy = torch.randn(T, in_f, generator=g).to(dtype), torch.randn(T, out_f, generator=g).to(dtype)
+    c, s = (torch.randn(out_f, k, generator=g) / k ** 0.5).to(dtype), torch.tensor([0.25]).to(dtype)
+    W = c.double() @ ops.sq5_gen_2d(in_f, k, 8).double().cpu().t()
+    R = ops.sq5_gen_1d(in_f * out_f, 8).double().cpu().view(out_f, in_f)
+    if rbias:
+        W = W + 0.25 * R
+    leaves = [t.cuda().requires_grad_() for t in ([x, c, s] if rbias else [x, c])]
+    d = hip._desc(T, in_f, out_f, leaves[1], in_f, 1, 8, dtype, 0)
+    kept = _lib.load().rdb_linear_kept_bytes(ctypes.byref(d))
+    assert kept >= 4 * T * k
+    y = ops.linear(leaves[0], leaves[1], in_f, out_f, in_f, 1, 8, leaves[2] if rbias else None, None)
+    assert "OneCall" in repr(y.grad_fn)
+    grads = torch.autograd.grad(y, leaves, dy.cuda(), retain_graph=True)
+    X, D = x.double(), dy.double()
+    dW = D.t() @ X
+    want = [D @ W, dW @ ops.sq5_gen_2d(in_f, k, 8).double().cpu()] + ([(dW * R).sum().view(1)] if rbias else [])
+    tol = 5e-6 if dtype == torch.float32 else 8e-3
+    assert _rel(y.detach(), X @ W.t()) < tol
+    for got, w in zip(grads, want):
+        size = w.norm() if got.numel() > 1 else (dW * R).norm()
+        assert got.dtype == dtype and float((got.double().cpu() - w).norm() / size) < tol
+    # one at a time: the others are not formed
+    for leaf, w in zip(leaves, grads):
+        alone, = torch.autograd.grad(y, [leaf], dy.cuda(), retain_graph=True)
+        assert float((alone.double() - w.double()).norm() / w.double().norm().clamp_min(1e-3)) < 2 * tol
+
+
+def test_not_kept():
+    L = _lib.load()
+
+    def kept(T, in_f, out_f, k, dtype):
+        c = torch.empty(out_f, k, dtype=dtype)
+        return L.rdb_linear_kept_bytes(ctypes.byref(hip._desc(T, in_f, out_f, c, in_f, 1, 8, dtype, 0)))
+
+    assert kept(31, 784, 256, 64, torch.float32) == 0 and kept(128, 784, 256, 64, torch.float32) == 128 * 64 * 4
+    assert kept(2000, 784, 256, 64, torch.float32) == 0          # has a projection state
+    assert kept(128, 16, 256, 64, torch.float32) == 0            # z more than twice x
+    assert kept(96, 1001, 999, 100, torch.bfloat16) == 0 and kept(97, 1001, 999, 100, torch.bfloat16) > 0
+    assert kept(4096, 1000, 1000, 104, torch.bfloat16) == 0      # multiples of 8: the bf16 kernels
+    assert kept(4096, 100, 999, 101, torch.bfloat16) == 0

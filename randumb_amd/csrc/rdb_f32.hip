@@ -230,17 +230,41 @@ int linear_dcoef_f32(float *dcoef, float *d_scale_bias, const void *dy, int64_t 
     return check_launch("f32_sum_scalars_kernel");
 }
 
+// ----------------------------------------------------------------------------------------------- or the few-token kernels
+// fp32 with k <= 64: where the kernels above are ahead of the vector-ALU kernels of rdb_smallk.hip.  Microseconds of one direction
+// (contraction over J, expansion to E columns), fitted to 252 measured calls (k 16, 32, 64; 32 to 1024 tokens; 128 -> 256 to
+// 4096 -> 11008): what it picks is 0.2 us behind the faster of the two on average.  The vector-ALU kernels' hash costs a wave 0.2 us a
+// coefficient whatever the tokens, and their time grows with the products; the matrix cores' grows with the contraction a
+// block walks through alone.  1024 tokens x 4096 -> 11008, k = 64: forward 134 -> 41 us, dx 93 -> 45; 128 tokens x 784 -> 256,
+// k = 64: 20.4 -> 18.8, 20.8 -> 15.8; k = 16 stays (10.5 against 16.2).
+static double few_token_us(const rdb_linear_desc *d)
+{
+    return 7.0 + 0.21 * d->k + (double)d->tokens * (d->in_f + d->out_f) * (1.7e-6 + 0.9e-7 * d->k);
+}
+static double f32_products_us(const rdb_linear_desc *d, bool dx)
+{
+    const int64_t J = dx ? d->out_f : d->in_f, E = dx ? d->in_f : d->out_f;
+    return (dx ? 11.7 : 11.0) + 0.0034 * std::min<int64_t>(J, 5200) + 0.04 * d->k + 0.5e-6 * d->tokens * E;
+}
+bool f32_products_first(const rdb_linear_desc *d, bool dx)
+{
+    return d->algo == RDB_ALGO_AUTO && d->act_dtype == RDB_F32 && d->coef_dtype == RDB_F32 && d->k <= 64 && d->tokens >= 32 &&
+           f32_products_us(d, dx) < few_token_us(d);
+}
+
 // ----------------------------------------------------------------------------------------------- z kept from forward to backward
 // For the layers that have no projection state of their own (bf16 with sizes that are not multiples of 8, fp32 in the few-token
 // regime): the forward pass leaves z = x . N^T, [tokens x k] in fp32, and the backward pass takes it from there instead of
-// projecting x again.  Only while that is at most twice the size of x, which the caller keeps too.  Few tokens (in fp32 below 32,
-// in bf16 up to 96) stay with the kernels of rdb_smallk.hip.  4097 tokens x 1001 -> 999, k = 100 in bf16, forward and backward:
+// projecting x again.  Only while that is at most twice the size of x, which the caller keeps too.  Few tokens (in bf16 up to 96,
+// in fp32 below 32 and where the vector-ALU kernels' three calls take less: their coefficient gradient projects x again, 5 us more
+// than their forward pass, against 10 here) stay with the kernels of rdb_smallk.hip.  4097 tokens x 1001 -> 999, k = 100 in bf16, forward and backward:
 // 122 -> 98 us; 128 tokens x 784 -> 256, k = 64 in fp32: 22.7 + 11.1 + 27.8 us of few-token kernels -> 17 + 6.
 int64_t linear_kept_f32_bytes(const rdb_linear_desc *d)
 {
     if (!fg_ok(d) || d->algo != RDB_ALGO_AUTO || d->tokens * std::max(d->in_f, d->out_f) >= (1ll << 28) || d->sO != d->in_f || d->sI != 1) return 0;
     const bool b16 = d->act_dtype == RDB_BF16;
     if (b16 ? (d->tokens <= 96 || !(d->in_f % 8 || d->out_f % 8 || d->k % 8) || d->k > d->in_f) : (d->tokens < 32 || d->k > 2 * d->in_f)) return 0;
+    if (!b16 && d->k <= 64 && f32_products_us(d, false) + f32_products_us(d, true) + 10.0 > 3.0 * few_token_us(d) + 5.0) return 0;
     return up256(d->tokens * d->k * 4);
 }
 

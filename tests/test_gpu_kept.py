@@ -59,3 +59,19 @@ def test_not_kept():
     assert kept(96, 1001, 999, 100, torch.bfloat16) == 0 and kept(97, 1001, 999, 100, torch.bfloat16) > 0
     assert kept(4096, 1000, 1000, 104, torch.bfloat16) == 0      # multiples of 8: the bf16 kernels
     assert kept(4096, 100, 999, 101, torch.bfloat16) == 0
+
+
+@pytest.mark.parametrize("T,in_f,out_f,k", [(32, 128, 256, 64), (33, 785, 257, 33), (300, 128, 256, 32), (1024, 1000, 3000, 17), (1023, 770, 12, 64)])
+def test_few_token_forward_and_dx_on_the_matrix_cores(T, in_f, out_f, k):
+    """fp32, k <= 64, on either side of the rule that chooses between the few-token kernels and the matrix cores, and without a
+    workspace (which leaves neither of them)."""
+    g = torch.Generator().manual_seed(T + k)
+    x, dy, c = torch.randn(T, in_f, generator=g), torch.randn(T, out_f, generator=g), torch.randn(out_f, k, generator=g) / k ** 0.5
+    W = c.double() @ ops.sq5_gen_2d(in_f, k, 8).double().cpu().t()
+    assert _rel(hip.linear_fwd(x.cuda(), c.cuda(), in_f, out_f, in_f, 1, 8), x.double() @ W.t()) < 5e-6
+    assert _rel(hip.linear_bwd_dx(dy.cuda(), c.cuda(), in_f, out_f, in_f, 1, 8), dy.double() @ W) < 5e-6
+    y, xc, cc = torch.empty(T, out_f, device="cuda"), x.cuda(), c.cuda()
+    d = hip._desc(T, in_f, out_f, cc, in_f, 1, 8, torch.float32, 0)
+    rc = _lib.load().rdb_linear_fwd(y.data_ptr(), out_f, xc.data_ptr(), in_f, cc.data_ptr(), None, None, ctypes.byref(d), None, 0,
+                                    torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and _rel(y, x.double() @ W.t()) < 5e-6

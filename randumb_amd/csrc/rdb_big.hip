@@ -3,6 +3,7 @@
 //   big_y_kernel    y[tok, o]  = sum_m z[tok, m] * C[o, m] (+ bias[o])          256 (o) x 256 (tok) tiles
 //   big_bwd_kernel  t[tok, m]  = sum_o dy[tok, o] * C[o, m]                       256 (m) x 128 (tok) tiles, and in the same launch
 //                   dC[o, m]   = sum_tok dy[tok, o] * z[tok, m]                   256 (o) x 256 (m) tiles over all tokens
+//   big_y_kernel    dx[tok, i] = sum_m t[tok, m] * N[m, i]                        256 (i) x 256 (tok) tiles, N from memory
 // z, z^T and C^T come from the projection state in fragment order (rdb_direct.hpp: ProjLayout).  One persistent block per
 // compute unit (rdb_big.hpp).  Replaces materialize() + dense product and MmBackward's two products
 // (src/rten_cpp/RandumbTensor.py:942-946, 979-990) for such layers, as the 128-wide kernels of rdb_factored.hip / rdb_dx.hip do
@@ -40,8 +41,11 @@ static bool enough_tiles(int64_t tiles, int num_cus)
 }
 
 // ----------------------------------------------------------------------------------------------- y = z . C^T
+// Also dx = t . N, with N^T [in_f x k] in the place of C and t row-major: a noise value of a 64 x 256 tile's product is hashed again
+// for every 256 tokens, and at k > 256 that, not the matrix cores, is what the product waits for (4096 tokens x 4096, k = 1024: 57 us
+// for 34 GFLOP).  Written once (in_f * k values, 4 us) and read back out of L2 the same product runs at this kernel's rate.
 struct BigYParams {
-    const bf16_t *zf;   // fragment order, rows = tokens (tok32 / 32 row blocks), kpad / 16 k-steps
+    const bf16_t *zf;   // FRAG: fragment order, rows = tokens (tok32 / 32 row blocks), kpad / 16 k-steps; else [tokens x k] row-major
     const bf16_t *coef;
     const bf16_t *bias;
     bf16_t *y;
@@ -54,13 +58,29 @@ struct BigYParams {
 // half tiles (256 output features x 128 tokens) instead, two blocks to a tile, so that no block idles through a whole tile.
 constexpr int BY_HALF = 128;
 
-template <bool BIAS> __global__ __launch_bounds__(256, 1) void big_y_kernel(BigYParams p)
+template <int ROWS, bool FRAG> struct BigTokens {   // z (or t): rows = tokens
+    typedef typename std::conditional<FRAG, FragOperand<ROWS, 64>, GlobalOperand<ROWS, 64, K_CONT>>::type Operand;
+    static __device__ __forceinline__ void set(Operand &pb, const BigYParams &p, int tok0)
+    {
+        if constexpr (FRAG) {
+            pb.src = p.zf;
+            pb.ksteps = p.kpad >> 4;
+            pb.nrb = p.tok32 >> 5;
+            pb.rb0 = tok0 >> 5;
+            pb.klim_steps = p.kpad >> 4;
+        } else {
+            pb = Operand{p.zf, (int64_t)p.k, tok0, p.tokens, p.k, (int64_t)p.tokens * p.k};
+        }
+    }
+};
+
+template <bool BIAS, bool FRAG = true> __global__ __launch_bounds__(256, 1) void big_y_kernel(BigYParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
     typedef GlobalOperand<BG, 64, K_CONT> PA;   // C: rows = output features
-    typedef FragOperand<BG, 64> PB;             // z: rows = tokens
-    typedef FragOperand<BY_HALF, 64> PH;        // z: the tokens of a half tile
+    typedef typename BigTokens<BG, FRAG>::Operand PB;
+    typedef typename BigTokens<BY_HALF, FRAG>::Operand PH;   // the tokens of a half tile
     const int total = p.tiles_o * p.tiles_t, vtotal = (total + 7) / 8 * 8, nblk = gridDim.x, nstage = (p.k + 63) / 64;
     const int full_rounds = vtotal / nblk, rest = vtotal - full_rounds * nblk;
     const bool halves = rest > 0 && 2 * rest <= nblk;
@@ -87,11 +107,7 @@ template <bool BIAS> __global__ __launch_bounds__(256, 1) void big_y_kernel(BigY
             int to, tt;
             big_y_decode(w, p.tiles_o, p.tiles_t, to, tt);
             init_a(to);
-            pb.src = p.zf;
-            pb.ksteps = p.kpad >> 4;
-            pb.nrb = p.tok32 >> 5;
-            pb.rb0 = tt * (BG / 32);
-            pb.klim_steps = p.kpad >> 4;
+            BigTokens<BG, FRAG>::set(pb, p, tt * BG);
             big_prefetch(regs, pa, pb, 0);
         };
         request(w);
@@ -129,11 +145,7 @@ template <bool BIAS> __global__ __launch_bounds__(256, 1) void big_y_kernel(BigY
         PH pb;
         BigRegs<PA, PH> regs;
         init_a(to);
-        pb.src = p.zf;
-        pb.ksteps = p.kpad >> 4;
-        pb.nrb = p.tok32 >> 5;
-        pb.rb0 = tok0 >> 5;
-        pb.klim_steps = p.kpad >> 4;
+        BigTokens<BY_HALF, FRAG>::set(pb, p, tok0);
         big_prefetch(regs, pa, pb, 0);
         f32x16 acc[BG / 64][BY_HALF / 64];
         big_zero<BG, BY_HALF>(acc);
@@ -159,7 +171,7 @@ struct BigBwdParams {
     const uint32_t *ctf_flag;
     const bf16_t *ztf;            // z transposed in fragment order (rows = coefficients)
     bf16_t *t;                    // [tokens x k] row-major
-    float *dc;                    // [out_f x k]: dcoef itself, or the partial-sum area a reduction adds to dcoef
+    void *dc;                     // [out_f x k], fp32 or bf16: dcoef itself, or the fp32 area a reduction adds to dcoef
     int tokens, out_f, k, kpad;
     int osteps, tsteps;           // k-steps per row block of ctf (out_f rounded up to 64, / 16) and of ztf (tokens likewise)
     int t_tiles_m, t_tiles_t;     // t tiles: 256 coefficients x 128 tokens; 0 tiles: the launch computes dC only
@@ -217,7 +229,7 @@ template <bool CT> __device__ __forceinline__ void big_t_items(const BigBwdParam
 }
 
 // dC tiles of one block, from the block's round r on; `base`: index of the first dC tile in the launch's list.
-__device__ __forceinline__ void big_dc_items(const BigBwdParams &p, bf16_t *lds, int &r, int base, int n2)
+template <typename E> __device__ __forceinline__ void big_dc_items(const BigBwdParams &p, bf16_t *lds, int &r, int base, int n2)
 {
     typedef GlobalOperand<BG, 64, M_CONT> PA;   // dy: rows = output features, contraction = tokens
     typedef FragOperand<BG, 64> PB;             // z^T: rows = coefficients
@@ -253,7 +265,7 @@ __device__ __forceinline__ void big_dc_items(const BigBwdParams &p, bf16_t *lds,
         const int wn = next();
         if (wn >= 0) request(wn);
         __builtin_amdgcn_sched_barrier(0);
-        big_store_f32<BG, BG>(acc, lds, p.dc, p.k, (int64_t)p.out_f * p.k, o0, p.out_f, m0, p.k, opaque_tid());
+        big_store_rows<BG, BG, E>(acc, lds, static_cast<E *>(p.dc), p.k, (int64_t)p.out_f * p.k, o0, p.out_f, m0, p.k, opaque_tid());
         if (wn < 0) break;
         w = wn;
     }
@@ -262,8 +274,10 @@ __device__ __forceinline__ void big_dc_items(const BigBwdParams &p, bf16_t *lds,
 // The launch's list holds the tiles of the longer kind first (a t tile contracts out_f with half-size stages, a dC tile the
 // tokens) and is dealt out to the blocks in rows of alternating direction (big_item): the blocks that got a long tile in
 // one row get the later, shorter ones of the next.  A block's rounds walk through the list in order, so it finishes its
-// tiles of the first kind before it starts on the second.
-__global__ __launch_bounds__(256, 1) void big_bwd_kernel(BigBwdParams p)
+// tiles of the first kind before it starts on the second.  E: dC's type.  A bf16 gradient leaves rounded from here: as fp32 sums
+// for the second launch to round it was 118 MB more through memory at 4096 -> 14336, k = 1024, and that launch waited for it
+// (125 us where its product takes 57).
+template <typename E> __global__ __launch_bounds__(256, 1) void big_bwd_kernel(BigBwdParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
@@ -275,9 +289,9 @@ __global__ __launch_bounds__(256, 1) void big_bwd_kernel(BigBwdParams p)
             if (ct) big_t_items<true>(p, lds, r, 0, n1);
             else big_t_items<false>(p, lds, r, 0, n1);
         }
-        if (n2) big_dc_items(p, lds, r, n1v, n2);
+        if (n2) big_dc_items<E>(p, lds, r, n1v, n2);
     } else {
-        if (n2) big_dc_items(p, lds, r, 0, n2);
+        if (n2) big_dc_items<E>(p, lds, r, 0, n2);
         if (n1) {
             if (ct) big_t_items<true>(p, lds, r, n2v, n1);
             else big_t_items<false>(p, lds, r, n2v, n1);
@@ -340,11 +354,58 @@ int linear_fwd_big(void *y, int64_t ldy, const void *state, const void *coef, co
     return launch_big(big_y_kernel<false>, p, p.tiles_o * p.tiles_t, num_cus, big_smem<BG, BG, TA, TB>(), s, "big_y_kernel");
 }
 
+// N^T[i, m] = noise(PRIME * i + m) as bf16, [in_f x k] row-major, k a multiple of 8: eight values a thread.  The rounded integers of the
+// kernels that hash into their operands, times 2^-31: a product with either has the same bits.
+__global__ __launch_bounds__(256) void noise_rows_bf16_kernel(bf16_t *__restrict__ out, uint32_t pieces, uint32_t k8, uint32_t seed)
+{
+    const uint32_t e = blockIdx.x * 256u + threadIdx.x;
+    if (e >= pieces) return;
+    const uint32_t i = e / k8, first = i * PN1 + (e - i * k8) * 8u * SQ5_N1 + seed;
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (float)(int32_t)sq5_tail(first + (uint32_t)j * SQ5_N1) * 4.656612873077392578125e-10f;
+    i32x4 h;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) h[j] = (int)f32x2_to_bf16x2(v[2 * j], v[2 * j + 1]);
+    *reinterpret_cast<i32x4 *>(out + (int64_t)e * 8) = h;
+}
+
+// Scratch for N^T where dx = t . N takes it from memory; 0: where it does not.
+int64_t dx_big_table_bytes(const rdb_linear_desc *d, int num_cus)
+{
+    const ProjLayout L = proj_layout(d);
+    if (!L.ok || L.fits_regs || d->in_f * d->k >= (1ll << 29) || !enough_tiles(cdiv(d->in_f, BG) * cdiv(d->tokens, BG), num_cus)) return 0;
+    return (d->in_f * d->k * (int64_t)sizeof(bf16_t) + 255) / 256 * 256;
+}
+
+// dx = t . N with t [tokens x k] row-major and room for N^T at `table`
+int linear_tn_big(void *dx, int64_t lddx, const void *t, void *table, const rdb_linear_desc *d, int num_cus, hipStream_t s)
+{
+    if (!dx_big_table_bytes(d, num_cus) || lddx % 8 || d->tokens * lddx >= (1ll << 29) || !big_aligned16(dx) || !big_aligned16(t) || !big_aligned16(table))
+        return RDB_E_UNSUPPORTED;
+    const uint32_t pieces = (uint32_t)(d->in_f * d->k / 8);
+    noise_rows_bf16_kernel<<<(unsigned)cdiv(pieces, 256), 256, 0, s>>>(static_cast<bf16_t *>(table), pieces, (uint32_t)(d->k / 8), d->seed);
+    if (int rc = check_launch("noise_rows_bf16_kernel")) return rc;
+    BigYParams p = {};
+    p.zf = static_cast<const bf16_t *>(t);
+    p.coef = static_cast<const bf16_t *>(table);
+    p.y = static_cast<bf16_t *>(dx);
+    p.ldy = lddx;
+    p.y_elems = (d->tokens - 1) * lddx + d->in_f;
+    p.tokens = (int)d->tokens;
+    p.out_f = (int)d->in_f;
+    p.k = (int)d->k;
+    p.tiles_o = (int)cdiv(d->in_f, BG);
+    p.tiles_t = (int)cdiv(d->tokens, BG);
+    typedef OperandTile<BG, 64, K_CONT> TA;
+    return launch_big(big_y_kernel<false, false>, p, p.tiles_o * p.tiles_t, num_cus, big_smem<BG, BG, TA, TA>(), s, "big_y_kernel (dx = t . N)");
+}
+
 // First launch of the backward pass: t (row-major, for the t . N kernel of the tile engine) and dC.  `dc`: where the
-// coefficient gradient's sums go (dcoef, or the area a reduction adds to dcoef).  want_t / want_dc: which of the two
+// coefficient gradient's sums go (dcoef, fp32 or, with dc_bf16, bf16; or the area a reduction adds to dcoef).  want_t / want_dc: which of the two
 // (t alone needs no state, dC alone no coefficients).
-int linear_bwd_big(void *t, float *dc, const void *dy, int64_t lddy, const void *state, const void *coef, const rdb_linear_desc *d, int num_cus,
-                   bool want_t, bool want_dc, hipStream_t s)
+int linear_bwd_big(void *t, void *dc, bool dc_bf16, const void *dy, int64_t lddy, const void *state, const void *coef, const rdb_linear_desc *d,
+                   int num_cus, bool want_t, bool want_dc, hipStream_t s)
 {
     const ProjLayout L = proj_layout(d);
     if (!L.ok || d->tokens * lddy >= (1ll << 29) || lddy % 8) return RDB_E_UNSUPPORTED;
@@ -376,7 +437,9 @@ int linear_bwd_big(void *t, float *dc, const void *dy, int64_t lddy, const void 
     constexpr size_t smem_dc = big_smem<BG, BG, TM, TF>(), smem_t = big_smem<BG, BT_TOK, TM, TD>();
     p.t_first = d->out_f >= 2 * d->tokens;   // stages of 64 at half the matrix work against stages of 64 over the tokens
     const int items = (p.t_tiles_m * p.t_tiles_t + 7) / 8 * 8 + (p.c_tiles_o * p.c_tiles_m + 7) / 8 * 8;
-    return launch_big(big_bwd_kernel, p, items, num_cus, smem_dc > smem_t ? smem_dc : smem_t, s, "big_bwd_kernel");
+    const size_t smem = smem_dc > smem_t ? smem_dc : smem_t;
+    if (dc_bf16) return launch_big(big_bwd_kernel<bf16_t>, p, items, num_cus, smem, s, "big_bwd_kernel<bf16>");
+    return launch_big(big_bwd_kernel<float>, p, items, num_cus, smem, s, "big_bwd_kernel");
 }
 
 }  // namespace rdb

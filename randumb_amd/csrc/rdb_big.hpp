@@ -298,22 +298,22 @@ __device__ __forceinline__ void big_store_bf16(f32x16 (&acc)[BM / 64][BN / 64], 
     __syncthreads();
 }
 
-// D[a][b] as fp32 to out[(a0 + a) * ld + b0 + b]: each wave passes its quadrant through an LDS patch of 32 rows x its
-// BN / 2 columns (row stride + 4 floats), so that a lane stores 16 bytes of a row.  Pieces outside na x nb are dropped by the
-// buffer bounds check.  `out` holds out_elems < 2^29 floats; nb, ld multiples of 4.  Non-temporal: the sums are for a later launch.
+// D[a][b] to out[(a0 + a) * ld + b0 + b], as fp32 or rounded to bf16: each wave passes its quadrant through an LDS patch of 32 rows x
+// its BN / 2 columns (row stride + 4 floats), so that a lane stores 16 bytes of a row.  Pieces outside na x nb are dropped by the
+// buffer bounds check.  `out` holds out_elems < 2^29 values; nb, ld multiples of 4 (bf16: 8).  Non-temporal: nothing here reads them.
 constexpr uint32_t BUFFER_OOB_ANY = 0xfffffff0u;   // outside a buffer of any size up to 2^32 - 16 bytes
-template <int BM, int BN>
-__device__ __forceinline__ void big_store_f32(f32x16 (&acc)[BM / 64][BN / 64], bf16_t *__restrict__ lds, float *__restrict__ out, int64_t ld,
-                                              int64_t out_elems, int a0, int na, int b0, int nb, int t)
+template <int BM, int BN, typename E>
+__device__ __forceinline__ void big_store_rows(f32x16 (&acc)[BM / 64][BN / 64], bf16_t *__restrict__ lds, E *__restrict__ out, int64_t ld,
+                                               int64_t out_elems, int a0, int na, int b0, int nb, int t)
 {
-    constexpr int MI = BM / 64, NI = BN / 64, COLS = NI * 32, LDP = COLS + 4;
+    constexpr int MI = BM / 64, NI = BN / 64, COLS = NI * 32, LDP = COLS + 4, PER = 16 / (int)sizeof(E);
     const int wave = t >> 6, lane = t & 63, r = lane & 31, g = lane >> 5, wm = wave >> 1, wn = wave & 1;
     float *patch = reinterpret_cast<float *>(lds) + wave * 32 * LDP;
     acc_settle<BM / 64, BN / 64>(acc);
-    constexpr int LPR = COLS / 4;                 // lanes per row of the patch
+    constexpr int LPR = COLS / PER;               // lanes per row of the patch
     constexpr int RPP = 64 / LPR;                 // rows per pass
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(out, 0, (int)(out_elems * 4), 0x00020000);
-    const int col = (lane % LPR) * 4, b = b0 + wn * COLS + col;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(out, 0, (int)(out_elems * (int)sizeof(E)), 0x00020000);
+    const int col = (lane % LPR) * PER, b = b0 + wn * COLS + col;
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi) {
 #pragma unroll
@@ -326,8 +326,16 @@ __device__ __forceinline__ void big_store_f32(f32x16 (&acc)[BM / 64][BN / 64], b
         for (int q = 0; q < 32 / RPP; ++q) {
             const int row = q * RPP + lane / LPR;
             const int a = a0 + wm * MI * 32 + mi * 32 + row;
-            const uint32_t off = (a < na && b < nb) ? (uint32_t)(((int64_t)a * ld + b) * 4) : BUFFER_OOB_ANY;
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, *reinterpret_cast<const f32x4 *>(patch + row * LDP + col)), rs, (int)off, 0, 2);
+            const uint32_t off = (a < na && b < nb) ? (uint32_t)(((int64_t)a * ld + b) * (int)sizeof(E)) : BUFFER_OOB_ANY;
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(patch + row * LDP + col);
+            if constexpr (sizeof(E) == 2) {
+                const f32x4 u = *reinterpret_cast<const f32x4 *>(patch + row * LDP + col + 4);
+                const i32x4 h = {(int)f32x2_to_bf16x2(v[0], v[1]), (int)f32x2_to_bf16x2(v[2], v[3]), (int)f32x2_to_bf16x2(u[0], u[1]),
+                                 (int)f32x2_to_bf16x2(u[2], u[3])};
+                __builtin_amdgcn_raw_buffer_store_b128(h, rs, (int)off, 0, 2);
+            } else {
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v), rs, (int)off, 0, 2);
+            }
         }
         __builtin_amdgcn_wave_barrier();
     }

@@ -339,8 +339,10 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
         BwdAParams a;
         const int dc_items = make_dc_params(a.dc, dcoef, dy, lddy, d, num_cus);
         dc_params_from_state(a.dc, z, d);
-        // one token range only: its sums are the result, stored straight into dcoef, and nothing is left to add up
-        const bool direct = a.dc.splits == 1 && !accumulate && !dc_bf16;
+        // one token range only (the 256-wide tiles always have one): its sums are the result, stored straight into dcoef, and
+        // nothing is left to add up
+        const bool big = big_bwd_applies(d, num_cus) && !tn_stationary_ok(d, lddx);
+        const bool direct = !accumulate && (big || (a.dc.splits == 1 && !dc_bf16));
         a.dc.partial = direct ? dcoef : reinterpret_cast<float *>(static_cast<char *>(workspace) + align256(linear_dx_factored_workspace(d)));
         a.dyc = p1;
         {   // the transposed coefficients, if the forward pass left them in the state (its header says so)
@@ -352,14 +354,13 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
         }
         if (tn_stationary_ok(d, lddx)) a.dyc.frag_ksteps = (int)cdiv(d->k, 64) * 4;   // the t.N kernel below keeps t in registers
         a.dc_blocks = xcd_grid_size(dc_items);
-        int rc = RDB_OK, red_splits = a.dc.splits;
+        int rc = RDB_OK;
+        const int red_splits = big ? 1 : a.dc.splits;
         if (!(g_bwd_parts & 1)) {
-            if (big_bwd_applies(d, num_cus) && !a.dyc.frag_ksteps) red_splits = 1;
-        } else if (big_bwd_applies(d, num_cus) && !a.dyc.frag_ksteps) {
+        } else if (big) {
             // long coefficient dimension and many tiles: both products on 256-wide tiles; a dC tile contracts all tokens, so
-            // there is one set of sums, stored where the first split's would go
-            rc = linear_bwd_big(workspace, a.dc.partial, dy, lddy, z, coef, d, num_cus, true, true, s);
-            red_splits = 1;
+            // there is one set of sums, stored into dcoef or, when it is to be added to, where the first split's would go
+            rc = linear_bwd_big(workspace, a.dc.partial, direct && dc_bf16, dy, lddy, z, coef, d, num_cus, true, true, s);
         } else {
             size_t smem = smem_dc > smem_dyc ? smem_dc : smem_dyc;
             if (int rl = reserve_lds(reinterpret_cast<const void *>(bwd_dc_dyc_kernel), smem, "bwd_dc_dyc_kernel")) return rl;
@@ -400,6 +401,11 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             default: bwd_tns_red_kernel<4><<<grid, block, smem_s, s>>>(bs); break;
             }
             return check_launch("bwd_tns_red_kernel");
+        }
+        const int64_t table = dx_big_table_bytes(d, num_cus), base = align256(linear_bwd_projected_workspace(d, num_cus, accumulate || dc_bf16));
+        if (direct && table && workspace_bytes >= base + table) {   // nothing to add up, and room for N^T
+            rc = linear_tn_big(dx, lddx, workspace, static_cast<char *>(workspace) + base, d, num_cus, s);
+            if (rc != RDB_E_UNSUPPORTED) return rc;
         }
         BwdBParams b;
         const int tn_items = make_tn_params(b.tn, dx, lddx, workspace, d);

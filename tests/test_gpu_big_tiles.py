@@ -231,3 +231,41 @@ def test_big_tiles_on_chunked_tokens(hip):
     assert torch.equal(outs[2][0], outs[0][0]) and torch.equal(outs[2][1], outs[0][1])
     assert rel_l2(outs[2][2].cpu().numpy(), outs[0][2].cpu().numpy()) < 1e-5
     assert float(outs[2][2].abs().sum()) > 0
+
+
+@pytest.mark.parametrize("T,in_f,out_f,k", [(300, 264, 512, 264), (128, 8, 264, 264), (2088, 1032, 520, 1000), (257, 520, 256, 328)])
+def test_backward_with_the_noise_from_memory(T, in_f, out_f, k):
+    """dx = t . N with N written once, and dC rounded to bf16 by the tiles themselves: the bits of the kernel that hashes and of the
+    launch that adds fp32 sums up; also with a workspace that has no room for N."""
+    import ctypes
+
+    from randumb_amd import _lib, hip, ops
+
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(k)
+    x, dy = torch.randn(T, in_f, generator=g).bfloat16().cuda(), torch.randn(T, out_f, generator=g).bfloat16().cuda()
+    c = (torch.randn(out_f, k, generator=g) / k ** 0.5).bfloat16().cuda()
+    d = hip._desc(T, in_f, out_f, c, in_f, 1, 5, torch.bfloat16, 0)
+    ref = ctypes.byref(d)
+    old = lib.rdb_set_big_tiles(2)
+    try:
+        y, state = hip.linear_project_fwd(x, c, 5)
+        full = lib.rdb_linear_workspace_bytes(4, ref)
+        table = -(-in_f * k * 2 // 256) * 256
+        results = []
+        for size, dtype in ((full, torch.bfloat16), (full - table, torch.bfloat16), (full, torch.float32)):
+            dx, dc = torch.empty_like(x), torch.empty(out_f, k, dtype=dtype, device="cuda")
+            ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+            rc = lib.rdb_linear_bwd_projected_to(dx.data_ptr(), in_f, dc.data_ptr(), 1 if dtype == torch.bfloat16 else 0, dy.data_ptr(), out_f,
+                                                 state.data_ptr(), c.data_ptr(), ref, ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream)
+            assert rc == 0
+            results.append((dx, dc))
+    finally:
+        lib.rdb_set_big_tiles(old)
+    for dx, dc in results[1:]:
+        assert torch.equal(dx, results[0][0]) and torch.equal(dc.bfloat16(), results[0][1])
+    N = ops.sq5_gen_2d(in_f, k, 5).float().cpu()
+    t = dy.float().cpu() @ c.float().cpu()
+    want_dx, want_dc = t @ N.t(), dy.float().cpu().t() @ (x.float().cpu() @ N)
+    for got, want in ((results[0][0], want_dx), (results[0][1], want_dc)):
+        assert float((got.float().cpu() - want).norm() / want.norm()) < 1e-2

@@ -3,6 +3,7 @@
 //   big_y_kernel    y[tok, o]  = sum_m z[tok, m] * C[o, m] (+ bias[o])          256 (o) x 256 (tok) tiles
 //   big_bwd_kernel  t[tok, m]  = sum_o dy[tok, o] * C[o, m]                       256 (m) x 128 (tok) tiles, and in the same launch
 //                   dC[o, m]   = sum_tok dy[tok, o] * z[tok, m]                   256 (o) x 256 (m) tiles over all tokens
+//   big_z_kernel    z[tok, m]  = sum_i x[tok, i] * N[m, i]                        256 (m) x 128 (tok) tiles, N from memory
 //   big_y_kernel    dx[tok, i] = sum_m t[tok, m] * N[m, i]                        256 (i) x 256 (tok) tiles, N from memory
 // z, z^T and C^T come from the projection state in fragment order (rdb_direct.hpp: ProjLayout).  One persistent block per
 // compute unit (rdb_big.hpp).  Replaces materialize() + dense product and MmBackward's two products
@@ -299,6 +300,116 @@ template <typename E> __global__ __launch_bounds__(256, 1) void big_bwd_kernel(B
     }
 }
 
+// ----------------------------------------------------------------------------------------------- z = x . N^T
+// For layers with as many tiles as half the compute units.  The kernel that hashes (factored_z_kernel) has 32 x 256 tiles: every noise
+// value hashed again for every 256 tokens, x read again for every 32 coefficients, 2 KB out of LDS per matrix instruction (4096 tokens x
+// 4096, k = 1024: 96 us for 34 GFLOP).  Blocks past the tiles transpose C for the backward pass, 64 x 256 of it at a time.
+struct BigZParams {
+    const bf16_t *noise;   // N [k x in_f]
+    const bf16_t *x;
+    int64_t ldx;
+    bf16_t *zf, *ztf;      // z and z^T in fragment order (ProjLayout)
+    uint32_t *flag;        // header of the state
+    const bf16_t *coef;    // NULL, or C [out_f x k], to leave transposed in ctf
+    bf16_t *ctf;
+    int tokens, in_f, out_f, k, kpad, tok32, tok64, out64;
+    int tiles_m, tiles_t, tile_blocks;
+};
+constexpr int BZ_TOK = 128;
+
+// 16 rows (the contraction) x 32 columns of an LDS matrix with row stride LD, as the fragment whose rows are those columns
+template <int LD> __device__ __forceinline__ f32x4 transposed_frag(const bf16_t *src, int lane)
+{
+    const int sl = lane & 15, qq = (lane >> 4) & 1, g = lane >> 5;
+    const bf16_t *p = src + (g * 8 + (sl >> 2)) * LD + qq * 16 + (sl & 3) * 4;
+    Frag8 f;
+    f.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)(p));
+    f.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)(p + 4 * LD));
+    return f.f4;
+}
+
+__device__ __forceinline__ void transpose_coef(const BigZParams &p, bf16_t *lds, int block, int nblocks)
+{
+    constexpr int LD = BG + 32;   // 64 bytes of padding: the four rows of a transposing read cover all banks
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, osteps = p.out64 >> 4, mt = (p.kpad + BG - 1) / BG;
+    for (int w = block; w < (p.out64 >> 6) * mt; w += nblocks) {
+        const int o0 = (w / mt) * 64, m0 = (w % mt) * BG;
+        f32x4 v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int o = o0 + q * 8 + (t >> 5), m = m0 + (t & 31) * 8;
+            v[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (o < p.out_f && m < p.k) v[q] = *reinterpret_cast<const f32x4 *>(p.coef + (int64_t)o * p.k + m);   // k is a multiple of 8
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) *reinterpret_cast<f32x4 *>(lds + (q * 8 + (t >> 5)) * LD + (t & 31) * 8) = v[q];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int mb = wave * 2 + (q >> 2), ks = q & 3;
+            const f32x4 f = transposed_frag<LD>(lds + ks * 16 * LD + mb * 32, lane);
+            if (m0 + mb * 32 < p.kpad)
+                store_stream(reinterpret_cast<f32x4 *>(p.ctf + ((int64_t)((m0 >> 5) + mb) * osteps + (o0 >> 4) + ks) * 512 + lane * 8), f);
+        }
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(256, 1) void big_z_kernel(BigZParams p)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
+    if ((int)blockIdx.x >= p.tile_blocks) {
+        transpose_coef(p, lds, (int)blockIdx.x - p.tile_blocks, (int)gridDim.x - p.tile_blocks);
+        return;
+    }
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, r = lane & 31, g = lane >> 5, wm = wave >> 1, wn = wave & 1;
+    if (blockIdx.x == 0 && t == 0) {
+        p.flag[0] = p.coef ? 1u : 0u;
+        p.flag[1] = 0u;
+    }
+    const int total = p.tiles_m * p.tiles_t, w = xcd_work_item(blockIdx.x, total);   // coefficient tile fastest: neighbours share the x tile
+    if (w >= total) return;
+    const int m0 = (w % p.tiles_m) * BG, tok0 = (w / p.tiles_m) * BZ_TOK;
+    typedef GlobalOperand<BG, 64, K_CONT> PA;
+    typedef GlobalOperand<BZ_TOK, 64, K_CONT> PB;
+    PA pa = {p.noise, (int64_t)p.in_f, m0, p.k, p.in_f, (int64_t)p.k * p.in_f};
+    PB pb = {p.x, p.ldx, tok0, p.tokens, p.in_f, (int64_t)(p.tokens - 1) * p.ldx + p.in_f};
+    BigRegs<PA, PB> regs;
+    big_prefetch(regs, pa, pb, 0);
+    constexpr int MI = BG / 64, NI = BZ_TOK / 64, LD = BG + 8;
+    f32x16 acc[MI][NI];
+    big_zero<BG, BZ_TOK>(acc);
+    big_mainloop<BG, BZ_TOK>(acc, lds, regs, pa, pb, (p.in_f + 63) / 64);
+    // D[a = coefficient][b = token] to LDS once, as bf16 rows of tokens; from there in both orders.  Coefficients past k and tokens
+    // past the end are zeros.
+    acc_settle<MI, NI>(acc);
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+            for (int jq = 0; jq < 4; ++jq)
+                store4<bf16_t>(lds + (wn * NI * 32 + ni * 32 + r) * LD + wm * MI * 32 + mi * 32 + 8 * jq + 4 * g, acc_read(acc[mi][ni][jq * 4 + 0]),
+                               acc_read(acc[mi][ni][jq * 4 + 1]), acc_read(acc[mi][ni][jq * 4 + 2]), acc_read(acc[mi][ni][jq * 4 + 3]));
+    __syncthreads();
+    const int ksteps = p.kpad >> 4, tsteps = p.tok64 >> 4;
+#pragma unroll
+    for (int q = 0; q < BG * BZ_TOK / 8 / 256; ++q) {   // rows = tokens: a piece is 8 coefficients of one token
+        const int idx = q * 256 + t, b = idx % BZ_TOK, a = (idx / BZ_TOK) * 8, gb = tok0 + b, ga = m0 + a;
+        if (gb < p.tok32 && ga < p.kpad)
+            *reinterpret_cast<f32x4 *>(p.zf + (((int64_t)(gb >> 5) * ksteps + (ga >> 4)) * 512 + (((ga >> 3) & 1) * 32 + (gb & 31)) * 8)) =
+                *reinterpret_cast<const f32x4 *>(lds + b * LD + a);
+    }
+#pragma unroll
+    for (int q = 0; q < BG / 32 * (BZ_TOK / 16) / 4; ++q) {   // rows = coefficients
+        const int u = wave * (BG / 32 * (BZ_TOK / 16) / 4) + q, mb = u / (BZ_TOK / 16), ks = u % (BZ_TOK / 16);
+        const f32x4 f = transposed_frag<LD>(lds + ks * 16 * LD + mb * 32, lane);
+        if (tok0 + ks * 16 < p.tok64 && m0 + mb * 32 < p.kpad)
+            store_stream(reinterpret_cast<f32x4 *>(p.ztf + ((int64_t)((m0 >> 5) + mb) * tsteps + (tok0 >> 4) + ks) * 512 + lane * 8), f);
+    }
+}
+
 // ----------------------------------------------------------------------------------------------- host side
 static bool big_aligned16(const void *q) { return ((uintptr_t)q & 15) == 0; }
 
@@ -354,20 +465,28 @@ int linear_fwd_big(void *y, int64_t ldy, const void *state, const void *coef, co
     return launch_big(big_y_kernel<false>, p, p.tiles_o * p.tiles_t, num_cus, big_smem<BG, BG, TA, TB>(), s, "big_y_kernel");
 }
 
-// N^T[i, m] = noise(PRIME * i + m) as bf16, [in_f x k] row-major, k a multiple of 8: eight values a thread.  The rounded integers of the
-// kernels that hash into their operands, times 2^-31: a product with either has the same bits.
-__global__ __launch_bounds__(256) void noise_rows_bf16_kernel(bf16_t *__restrict__ out, uint32_t pieces, uint32_t k8, uint32_t seed)
+// The noise as bf16, rows of 8 * k8 values: value (r, c) with first-round value r * row_step + c * col_step + seed.  Eight values a
+// thread.  The rounded integers of the kernels that hash into their operands, times 2^-31: a product with either has the same bits.
+__global__ __launch_bounds__(256) void noise_rows_bf16_kernel(bf16_t *__restrict__ out, uint32_t pieces, uint32_t k8, uint32_t row_step, uint32_t col_step,
+                                                              uint32_t seed)
 {
     const uint32_t e = blockIdx.x * 256u + threadIdx.x;
     if (e >= pieces) return;
-    const uint32_t i = e / k8, first = i * PN1 + (e - i * k8) * 8u * SQ5_N1 + seed;
+    const uint32_t r = e / k8, first = r * row_step + (e - r * k8) * 8u * col_step + seed;
     float v[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = (float)(int32_t)sq5_tail(first + (uint32_t)j * SQ5_N1) * 4.656612873077392578125e-10f;
+    for (int j = 0; j < 8; ++j) v[j] = (float)(int32_t)sq5_tail(first + (uint32_t)j * col_step) * 4.656612873077392578125e-10f;
     i32x4 h;
 #pragma unroll
     for (int j = 0; j < 4; ++j) h[j] = (int)f32x2_to_bf16x2(v[2 * j], v[2 * j + 1]);
     *reinterpret_cast<i32x4 *>(out + (int64_t)e * 8) = h;
+}
+// rows x cols values, cols a multiple of 8, fewer than 2^29
+static int launch_noise_rows(void *out, int64_t rows, int64_t cols, uint32_t row_step, uint32_t col_step, uint32_t seed, hipStream_t s)
+{
+    const uint32_t pieces = (uint32_t)(rows * cols / 8);
+    noise_rows_bf16_kernel<<<(unsigned)cdiv(pieces, 256), 256, 0, s>>>(static_cast<bf16_t *>(out), pieces, (uint32_t)(cols / 8), row_step, col_step, seed);
+    return check_launch("noise_rows_bf16_kernel");
 }
 
 // Scratch for N^T where dx = t . N takes it from memory; 0: where it does not.
@@ -383,9 +502,7 @@ int linear_tn_big(void *dx, int64_t lddx, const void *t, void *table, const rdb_
 {
     if (!dx_big_table_bytes(d, num_cus) || lddx % 8 || d->tokens * lddx >= (1ll << 29) || !big_aligned16(dx) || !big_aligned16(t) || !big_aligned16(table))
         return RDB_E_UNSUPPORTED;
-    const uint32_t pieces = (uint32_t)(d->in_f * d->k / 8);
-    noise_rows_bf16_kernel<<<(unsigned)cdiv(pieces, 256), 256, 0, s>>>(static_cast<bf16_t *>(table), pieces, (uint32_t)(d->k / 8), d->seed);
-    if (int rc = check_launch("noise_rows_bf16_kernel")) return rc;
+    if (int rc = launch_noise_rows(table, d->in_f, d->k, PN1, SQ5_N1, d->seed, s)) return rc;   // N^T[i, m] = noise(PRIME * i + m)
     BigYParams p = {};
     p.zf = static_cast<const bf16_t *>(t);
     p.coef = static_cast<const bf16_t *>(table);
@@ -399,6 +516,47 @@ int linear_tn_big(void *dx, int64_t lddx, const void *t, void *table, const rdb_
     p.tiles_t = (int)cdiv(d->tokens, BG);
     typedef OperandTile<BG, 64, K_CONT> TA;
     return launch_big(big_y_kernel<false, false>, p, p.tiles_o * p.tiles_t, num_cus, big_smem<BG, BG, TA, TA>(), s, "big_y_kernel (dx = t . N)");
+}
+
+// state <- z (and C transposed, with coef), N in `room` (room_bytes of it; the rows of the forward product to come will do)
+int linear_z_big(void *state, const void *x, int64_t ldx, const void *coef, void *room, int64_t room_bytes, const rdb_linear_desc *d, int num_cus,
+                 hipStream_t s)
+{
+    const ProjLayout L = proj_layout(d);
+    const int64_t tiles = cdiv(d->k, BG) * cdiv(d->tokens, BZ_TOK);
+    if (!L.ok || L.fits_regs || !enough_tiles(tiles, num_cus) || d->in_f * d->k >= (1ll << 29) || !room || room_bytes < d->in_f * d->k * 2)
+        return RDB_E_UNSUPPORTED;
+    if (ldx % 8 || d->tokens * ldx >= (1ll << 29) || !big_aligned16(x) || !big_aligned16(state) || !big_aligned16(coef) || !big_aligned16(room))
+        return RDB_E_UNSUPPORTED;
+    if (int rc = launch_noise_rows(room, d->k, d->in_f, SQ5_N1, PN1, d->seed, s)) return rc;   // N[m, i] = noise(PRIME * i + m)
+    char *st = static_cast<char *>(state);
+    BigZParams p;
+    p.noise = static_cast<const bf16_t *>(room);
+    p.x = static_cast<const bf16_t *>(x);
+    p.ldx = ldx;
+    p.zf = reinterpret_cast<bf16_t *>(st + L.zf_off);
+    p.ztf = reinterpret_cast<bf16_t *>(st + L.ztf_off);
+    p.flag = reinterpret_cast<uint32_t *>(st);
+    p.coef = static_cast<const bf16_t *>(coef);
+    p.ctf = reinterpret_cast<bf16_t *>(st + L.ctf_off);
+    p.tokens = (int)d->tokens;
+    p.in_f = (int)d->in_f;
+    p.out_f = (int)d->out_f;
+    p.k = (int)d->k;
+    p.kpad = L.kpad;
+    p.tok32 = (int)L.tok32;
+    p.tok64 = (int)L.tok64;
+    p.out64 = (int)L.out64;
+    p.tiles_m = (int)cdiv(d->k, BG);
+    p.tiles_t = (int)cdiv(d->tokens, BZ_TOK);
+    p.tile_blocks = xcd_grid_size((int)tiles);
+    const size_t smem = big_smem<BG, BZ_TOK, OperandTile<BG, 64, K_CONT>, OperandTile<BZ_TOK, 64, K_CONT>>();
+    if (int rl = reserve_lds(reinterpret_cast<const void *>(big_z_kernel), smem, "big_z_kernel")) return rl;
+    // the transposing blocks: the compute units that the tiles leave free, or as many as there are
+    int c_blocks = coef ? num_cus - p.tile_blocks : 0;
+    if (coef && c_blocks < num_cus / 4) c_blocks = num_cus;
+    big_z_kernel<<<p.tile_blocks + c_blocks, 256, smem, s>>>(p);
+    return check_launch("big_z_kernel");
 }
 
 // First launch of the backward pass: t (row-major, for the t . N kernel of the tile engine) and dC.  `dc`: where the

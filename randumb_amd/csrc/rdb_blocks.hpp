@@ -224,6 +224,8 @@ bool big_bwd_applies(const rdb_linear_desc *d, int num_cus);
 int linear_fwd_big(void *y, int64_t ldy, const void *state, const void *coef, const void *bias, const rdb_linear_desc *d, int num_cus, hipStream_t s);
 int linear_bwd_big(void *t, void *dc, bool dc_bf16, const void *dy, int64_t lddy, const void *state, const void *coef, const rdb_linear_desc *d,
                    int num_cus, bool want_t, bool want_dc, hipStream_t s);
+int linear_z_big(void *state, const void *x, int64_t ldx, const void *coef, void *room, int64_t room_bytes, const rdb_linear_desc *d, int num_cus,
+                 hipStream_t s);
 int64_t dx_big_table_bytes(const rdb_linear_desc *d, int num_cus);
 int linear_tn_big(void *dx, int64_t lddx, const void *t, void *table, const rdb_linear_desc *d, int num_cus, hipStream_t s);
 void set_big_tiles_mode(int mode);

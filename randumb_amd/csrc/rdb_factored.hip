@@ -521,7 +521,11 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
         // check the second call's conditions before the first launch, so that a refusal leaves nothing half done
         if (d->coef_dtype != RDB_BF16 || ldy % 8 || !aligned16(y) || !aligned16(coef)) return RDB_E_UNSUPPORTED;
         if (((uintptr_t)bias & 7) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
-        if (int rc = launch_z(state, x, ldx, with_ct ? coef : nullptr, y, ldy, d, s)) return rc;
+        // y's rows, contiguous and written last, hold N meanwhile; with a contraction in several ranges the sums differ (z_ranges)
+        const int64_t room = ldy == d->out_f && p.z.ranges == 1 ? d->tokens * d->out_f * (int64_t)sizeof(bf16_t) : 0;
+        int rc = linear_z_big(state, x, ldx, with_ct ? coef : nullptr, y, room, d, num_cus, s);
+        if (rc == RDB_E_UNSUPPORTED) rc = launch_z(state, x, ldx, with_ct ? coef : nullptr, y, ldy, d, s);
+        if (rc) return rc;
         return linear_fwd_projected(y, ldy, state, coef, bias, d, num_cus, s);
     }
     const ProjLayout L = proj_layout(d);

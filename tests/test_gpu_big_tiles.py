@@ -269,3 +269,21 @@ def test_backward_with_the_noise_from_memory(T, in_f, out_f, k):
     want_dx, want_dc = t @ N.t(), dy.float().cpu().t() @ (x.float().cpu() @ N)
     for got, want in ((results[0][0], want_dx), (results[0][1], want_dc)):
         assert float((got.float().cpu() - want).norm() / want.norm()) < 1e-2
+
+
+@pytest.mark.parametrize("T,in_f,out_f,k", [(300, 128, 264, 512), (1000, 200, 520, 328), (129, 1032, 2056, 264), (2088, 264, 4104, 1024), (32, 72, 1096, 264)])
+def test_projection_with_the_noise_from_memory(hip, T, in_f, out_f, k):
+    """z, z^T and C^T of the call that also forms y (256-wide tiles, N in y's rows) against those of the projection on its own (the kernel
+    that hashes): the same bits in everything computed from them, and in the state's pieces where nothing is padding."""
+    x, dy, coef, bias = [t.cuda() for t in _inputs(T, in_f, out_f, k, 3)]
+    want = _run(hip, 0, x, dy, coef, bias, in_f, out_f, k, 3, True)
+    before = hip.set_big_tiles(2)
+    try:
+        y, state = hip.linear_project_fwd(x, coef, 3, bias=bias)
+        alone = hip.linear_project(x, k, out_f, 3, coef=coef)
+        dx, dc = hip.linear_bwd_projected(dy, state, coef, in_f, 3)
+        dx_alone, dc_alone = hip.linear_bwd_projected(dy, alone, coef, in_f, 3)
+        torch.cuda.synchronize()
+    finally:
+        hip.set_big_tiles(before)
+    assert torch.equal(y, want[0]) and torch.equal(dx, want[1]) and torch.equal(dx, dx_alone) and torch.equal(dc, dc_alone)

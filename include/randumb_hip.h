@@ -173,7 +173,7 @@ enum {
 
 enum { RDB_OP_LINEAR_FWD = 0, RDB_OP_LINEAR_BWD_DX = 1, RDB_OP_LINEAR_BWD_DCOEF = 2, RDB_OP_LINEAR_BWD_PROJECTED = 3,
        RDB_OP_LINEAR_BWD_PROJECTED_TO = 4, RDB_OP_LINEAR_BWD_DX_DSCALE = 5, RDB_OP_LINEAR_RBIAS_BWD = 6,
-       RDB_OP_LINEAR_BWD_KEPT = 7 };
+       RDB_OP_LINEAR_BWD_KEPT = 7, RDB_OP_LINEAR_RBIAS_FWD = 8 };
 
 /* Device scratch (bytes) that entry point `op` can use for `desc`; 0 when it has no use for any.  A NULL or too small
  * workspace is never an error with RDB_ALGO_AUTO: the library then runs a kernel that needs none. */
@@ -227,6 +227,10 @@ int rdb_linear_bwd_dx_dscale(void *dx, int64_t lddx, float *d_scale_bias, const 
  * RDB_E_UNSUPPORTED and nothing launched otherwise.  Sums in a fixed order: the same bits from run to run. */
 int rdb_linear_rbias_fwd(void *y, int64_t ldy, const void *x, int64_t ldx, const void *scale_bias,
                          const rdb_linear_desc *desc, void *stream);
+/* The same with scratch for R (rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_FWD) bytes, 16-byte aligned; less, or NULL: R is hashed
+ * as the product needs it).  rdb_linear_rbias_bwd finds that scratch behind its sums. */
+int rdb_linear_rbias_fwd_ws(void *y, int64_t ldy, const void *x, int64_t ldx, const void *scale_bias, const rdb_linear_desc *desc,
+                            void *workspace, int64_t workspace_bytes, void *stream);
 int rdb_linear_rbias_bwd(void *dx, int64_t lddx, float *d_scale_bias, const void *dy, int64_t lddy, const void *x,
                          int64_t ldx, const void *scale_bias, const rdb_linear_desc *desc, void *workspace,
                          int64_t workspace_bytes, void *stream);

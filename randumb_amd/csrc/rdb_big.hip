@@ -4,6 +4,7 @@
 //   big_bwd_kernel  t[tok, m]  = sum_o dy[tok, o] * C[o, m]                       256 (m) x 128 (tok) tiles, and in the same launch
 //                   dC[o, m]   = sum_tok dy[tok, o] * z[tok, m]                   256 (o) x 256 (m) tiles over all tokens
 //   big_z_kernel    z[tok, m]  = sum_i x[tok, i] * N[m, i]                        256 (m) x 128 (tok) tiles, N from memory
+//   big_rbias_kernel  y += s * x . R^T,  dx += s * dy . R (any k)                 256 (features) x 128 (tok) tiles, R from memory
 //   big_y_kernel    dx[tok, i] = sum_m t[tok, m] * N[m, i]                        256 (i) x 256 (tok) tiles, N from memory
 // z, z^T and C^T come from the projection state in fragment order (rdb_direct.hpp: ProjLayout).  One persistent block per
 // compute unit (rdb_big.hpp).  Replaces materialize() + dense product and MmBackward's two products
@@ -41,10 +42,20 @@ static bool enough_tiles(int64_t tiles, int num_cus)
     return mode == 2 || (mode == 1 && tiles * 2 >= num_cus);
 }
 
+// Rows row0 .. of a [rows x cols] matrix in fragment order, rows padded to 32 and columns to 64
+template <int ROWS> __device__ __forceinline__ void frag_rows(FragOperand<ROWS, 64> &op, const bf16_t *src, int rows, int cols, int row0)
+{
+    op.src = src;
+    op.ksteps = ((cols + 63) >> 6) * 4;
+    op.nrb = (rows + 31) >> 5;
+    op.rb0 = row0 >> 5;
+    op.klim_steps = op.ksteps;
+}
+
 // ----------------------------------------------------------------------------------------------- y = z . C^T
-// Also dx = t . N, with N^T [in_f x k] in the place of C and t row-major: a noise value of a 64 x 256 tile's product is hashed again
+// Also dx = t . N, with N^T [in_f x k] in fragment order in the place of C and t row-major: a noise value of a 64 x 256 tile's product is hashed again
 // for every 256 tokens, and at k > 256 that, not the matrix cores, is what the product waits for (4096 tokens x 4096, k = 1024: 57 us
-// for 34 GFLOP).  Written once (in_f * k values, 4 us) and read back out of L2 the same product runs at this kernel's rate.
+// for 34 GFLOP).  Written once (in_f * k values, 6 us) and read back the same product takes 39.
 struct BigYParams {
     const bf16_t *zf;   // FRAG: fragment order, rows = tokens (tok32 / 32 row blocks), kpad / 16 k-steps; else [tokens x k] row-major
     const bf16_t *coef;
@@ -79,7 +90,7 @@ template <bool BIAS, bool FRAG = true> __global__ __launch_bounds__(256, 1) void
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
-    typedef GlobalOperand<BG, 64, K_CONT> PA;   // C: rows = output features
+    typedef typename std::conditional<FRAG, GlobalOperand<BG, 64, K_CONT>, FragOperand<BG, 64>>::type PA;   // C (N^T): rows = output features
     typedef typename BigTokens<BG, FRAG>::Operand PB;
     typedef typename BigTokens<BY_HALF, FRAG>::Operand PH;   // the tokens of a half tile
     const int total = p.tiles_o * p.tiles_t, vtotal = (total + 7) / 8 * 8, nblk = gridDim.x, nstage = (p.k + 63) / 64;
@@ -99,7 +110,10 @@ template <bool BIAS, bool FRAG = true> __global__ __launch_bounds__(256, 1) void
         return -1;
     };
     PA pa;
-    auto init_a = [&](int to) { pa = PA{p.coef, (int64_t)p.k, to * BG, p.out_f, p.k, (int64_t)p.out_f * p.k}; };
+    auto init_a = [&](int to) {
+        if constexpr (FRAG) pa = PA{p.coef, (int64_t)p.k, to * BG, p.out_f, p.k, (int64_t)p.out_f * p.k};
+        else frag_rows(pa, p.coef, p.out_f, p.k, to * BG);
+    };
     int w = next();
     if (w >= 0) {
         PB pb;
@@ -305,7 +319,7 @@ template <typename E> __global__ __launch_bounds__(256, 1) void big_bwd_kernel(B
 // value hashed again for every 256 tokens, x read again for every 32 coefficients, 2 KB out of LDS per matrix instruction (4096 tokens x
 // 4096, k = 1024: 96 us for 34 GFLOP).  Blocks past the tiles transpose C for the backward pass, 64 x 256 of it at a time.
 struct BigZParams {
-    const bf16_t *noise;   // N [k x in_f]
+    const bf16_t *noise;   // N [k x in_f] in fragment order
     const bf16_t *x;
     int64_t ldx;
     bf16_t *zf, *ztf;      // z and z^T in fragment order (ProjLayout)
@@ -371,9 +385,10 @@ __global__ __launch_bounds__(256, 1) void big_z_kernel(BigZParams p)
     const int total = p.tiles_m * p.tiles_t, w = xcd_work_item(blockIdx.x, total);   // coefficient tile fastest: neighbours share the x tile
     if (w >= total) return;
     const int m0 = (w % p.tiles_m) * BG, tok0 = (w / p.tiles_m) * BZ_TOK;
-    typedef GlobalOperand<BG, 64, K_CONT> PA;
+    typedef FragOperand<BG, 64> PA;
     typedef GlobalOperand<BZ_TOK, 64, K_CONT> PB;
-    PA pa = {p.noise, (int64_t)p.in_f, m0, p.k, p.in_f, (int64_t)p.k * p.in_f};
+    PA pa;
+    frag_rows(pa, p.noise, p.k, p.in_f, m0);
     PB pb = {p.x, p.ldx, tok0, p.tokens, p.in_f, (int64_t)(p.tokens - 1) * p.ldx + p.in_f};
     BigRegs<PA, PB> regs;
     big_prefetch(regs, pa, pb, 0);
@@ -407,6 +422,135 @@ __global__ __launch_bounds__(256, 1) void big_z_kernel(BigZParams p)
         const f32x4 f = transposed_frag<LD>(lds + ks * 16 * LD + mb * 32, lane);
         if (tok0 + ks * 16 < p.tok64 && m0 + mb * 32 < p.kpad)
             store_stream(reinterpret_cast<f32x4 *>(p.ztf + ((int64_t)((m0 >> 5) + mb) * tsteps + (tok0 >> 4) + ks) * 512 + lane * 8), f);
+    }
+}
+
+// ----------------------------------------------------------------------------------------------- out += s * src . R^T (or R)
+// The fused random bias's share (rdb_rbias.hip) with R written once as bf16 and read back.  Hashed into the product it costs its hash
+// for every 512 tokens on tiles of 64 features: 75 us for 38.6 GFLOP in either direction at 8192 tokens x 768 -> 3072; here 63 forward
+// (three tiles a block, each with 128 KB of dst to read and write) and 50 backward (one tile of 48 stages a block), and 5 for R.  Tiles
+// of 256 features x 128 tokens, so that 768 features still give 192 of them; one persistent block a compute unit.  What the epilogue
+// adds to is requested before a tile's main loop, the next tile's first stages before its epilogue.
+struct BigRBiasParams {
+    const bf16_t *noise;    // [cols x contraction] in fragment order
+    const bf16_t *src;      // [tokens x contraction]
+    bf16_t *dst;            // [tokens x cols]
+    const bf16_t *scale;    // one value
+    const bf16_t *other;    // DOT: [tokens x cols], what the product without s is reduced against: one sum a tile, in tile order
+    float *dot_part;
+    int64_t ld_src, ld_dst, ld_other;
+    int tokens, cols, contraction, tiles_a, tiles_t;
+};
+constexpr int BR_TOK = 128;
+
+template <bool DOT> __global__ __launch_bounds__(256, 1) void big_rbias_kernel(BigRBiasParams p)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
+    typedef FragOperand<BG, 64> PA;                 // R: rows = columns of dst
+    typedef GlobalOperand<BR_TOK, 64, K_CONT> PB;   // src: rows = tokens
+    constexpr int MI = BG / 64, NI = BR_TOK / 64, LDP = BG / 2 + 4;
+    const int total = p.tiles_a * p.tiles_t, vtotal = (total + 7) / 8 * 8, nblk = gridDim.x, nstage = (p.contraction + 63) / 64;
+    int rd = 0;
+    auto next = [&]() {
+        for (; rd * nblk + (int)blockIdx.x < vtotal; ++rd) {
+            const int w = xcd_work_item(rd * nblk + (int)blockIdx.x, total);
+            if (w < total) { ++rd; return w; }
+        }
+        return -1;
+    };
+    PA pa;
+    PB pb;
+    BigRegs<PA, PB> regs;
+    auto request = [&](int w) {   // feature tile fastest: neighbours share the tokens
+        frag_rows(pa, p.noise, p.cols, p.contraction, (w % p.tiles_a) * BG);
+        pb = PB{p.src, p.ld_src, (w / p.tiles_a) * BR_TOK, p.tokens, p.contraction, (int64_t)(p.tokens - 1) * p.ld_src + p.contraction};
+        big_prefetch(regs, pa, pb, 0);
+    };
+    int w = next();
+    if (w < 0) return;
+    request(w);
+    const float sval = bf16_to_f32(*p.scale);
+    const __amdgpu_buffer_rsrc_t rs_d = __builtin_amdgcn_make_buffer_rsrc(p.dst, 0, (int)(((int64_t)(p.tokens - 1) * p.ld_dst + p.cols) * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rs_o =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(DOT ? p.other : p.dst), 0, DOT ? (int)(((int64_t)(p.tokens - 1) * p.ld_other + p.cols) * 2) : 0, 0x00020000);
+    while (true) {
+        const int a0 = (w % p.tiles_a) * BG, tok0 = (w / p.tiles_a) * BR_TOK;
+        // the thread's pieces of the tile: 8 features of a token; 16 lanes cover a wave's 128 features
+        auto at = [&](int t, int ni, int q, int64_t ld) {
+            const int wave = t >> 6, lane = t & 63, tok = tok0 + (wave & 1) * NI * 32 + ni * 32 + q * 4 + (lane >> 4);
+            const int a = a0 + (wave >> 1) * MI * 32 + (lane & 15) * 8;   // cols is a multiple of 8: a piece lies inside or outside
+            return tok < p.tokens && a < p.cols ? (uint32_t)(((int64_t)tok * ld + a) * 2) : BUFFER_OOB;
+        };
+        Frag8 old[NI][8];
+        {
+            const int t = opaque_tid();
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    old[ni][q].f4 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_d, (int)at(t, ni, q, p.ld_dst), 0, 0));
+        }
+        f32x16 acc[MI][NI];
+        big_zero<BG, BR_TOK>(acc);
+        big_mainloop<BG, BR_TOK>(acc, lds, regs, pa, pb, nstage);
+        const int wn = next();
+        if (wn >= 0) request(wn);
+        __builtin_amdgcn_sched_barrier(0);
+        acc_settle<MI, NI>(acc);
+        const int t = opaque_tid(), wave = t >> 6, lane = t & 63, r = lane & 31, g = lane >> 5;
+        float *patch = reinterpret_cast<float *>(lds) + wave * 32 * LDP;   // 32 tokens x the wave's 128 features
+        float dot = 0.0f;
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) {
+            Frag8 ot[8];
+            if (DOT) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) ot[q].f4 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_o, (int)at(t, ni, q, p.ld_other), 0, 0));
+            }
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+                for (int jq = 0; jq < 4; ++jq)
+                    *reinterpret_cast<f32x4 *>(patch + r * LDP + mi * 32 + 8 * jq + 4 * g) =
+                        f32x4{acc_read(acc[mi][ni][jq * 4]), acc_read(acc[mi][ni][jq * 4 + 1]), acc_read(acc[mi][ni][jq * 4 + 2]), acc_read(acc[mi][ni][jq * 4 + 3])};
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_wave_barrier();   // LDS serves a wave's instructions in order: the reads see these writes
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const float *src = patch + (q * 4 + (lane >> 4)) * LDP + (lane & 15) * 8;
+                const f32x4 lo = *reinterpret_cast<const f32x4 *>(src), hi = *reinterpret_cast<const f32x4 *>(src + 4);
+                const uint32_t off = at(t, ni, q, p.ld_dst);
+                if (DOT) {   // outside the matrix `ot` reads as zeros
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        dot = fmaf(lo[2 * e], __uint_as_float(ot[q].u[e] << 16), dot);
+                        dot = fmaf(lo[2 * e + 1], __uint_as_float(ot[q].u[e] & 0xffff0000u), dot);
+                        dot = fmaf(hi[2 * e], __uint_as_float(ot[q].u[2 + e] << 16), dot);
+                        dot = fmaf(hi[2 * e + 1], __uint_as_float(ot[q].u[2 + e] & 0xffff0000u), dot);
+                    }
+                }
+                const Frag8 o = old[ni][q];
+                const i32x4 nw = {(int)f32x2_to_bf16x2(__uint_as_float(o.u[0] << 16) + sval * lo[0], __uint_as_float(o.u[0] & 0xffff0000u) + sval * lo[1]),
+                                  (int)f32x2_to_bf16x2(__uint_as_float(o.u[1] << 16) + sval * lo[2], __uint_as_float(o.u[1] & 0xffff0000u) + sval * lo[3]),
+                                  (int)f32x2_to_bf16x2(__uint_as_float(o.u[2] << 16) + sval * hi[0], __uint_as_float(o.u[2] & 0xffff0000u) + sval * hi[1]),
+                                  (int)f32x2_to_bf16x2(__uint_as_float(o.u[3] << 16) + sval * hi[2], __uint_as_float(o.u[3] & 0xffff0000u) + sval * hi[3])};
+                __builtin_amdgcn_raw_buffer_store_b128(nw, rs_d, (int)off, 0, 0);
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();   // the patches lie where the next tile's first stage goes
+        if (DOT) {   // lanes, then waves, in a fixed order
+            float *wsum = reinterpret_cast<float *>(lds);
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) dot += __shfl_xor(dot, o, 64);
+            if (lane == 0) wsum[wave] = dot;
+            __syncthreads();
+            if (t == 0) p.dot_part[w] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+            __syncthreads();
+        }
+        if (wn < 0) break;
+        w = wn;
     }
 }
 
@@ -465,36 +609,43 @@ int linear_fwd_big(void *y, int64_t ldy, const void *state, const void *coef, co
     return launch_big(big_y_kernel<false>, p, p.tiles_o * p.tiles_t, num_cus, big_smem<BG, BG, TA, TB>(), s, "big_y_kernel");
 }
 
-// The noise as bf16, rows of 8 * k8 values: value (r, c) with first-round value r * row_step + c * col_step + seed.  Eight values a
-// thread.  The rounded integers of the kernels that hash into their operands, times 2^-31: a product with either has the same bits.
-__global__ __launch_bounds__(256) void noise_rows_bf16_kernel(bf16_t *__restrict__ out, uint32_t pieces, uint32_t k8, uint32_t row_step, uint32_t col_step,
-                                                              uint32_t seed)
+// The noise as bf16 in fragment order (FragOperand): value (r, c) with first-round value r * row_step + c * col_step + seed, zeros for
+// rows and columns that are padding.  Eight values a thread.  The rounded integers of the kernels that hash into their operands, times
+// 2^-31: a product with either has the same bits.  Fragment order, because a stage of 64 columns then is consecutive kilobytes, not 128
+// bytes of each of 256 rows (4096 tokens x 4096, k = 1024, rows of 8 KB: z 66 -> 62 us; dx, rows of 2 KB: the same).
+__global__ __launch_bounds__(256) void noise_frag_bf16_kernel(bf16_t *__restrict__ out, uint32_t pieces, uint32_t ksteps, uint32_t rows, uint32_t cols,
+                                                              uint32_t row_step, uint32_t col_step, uint32_t seed)
 {
     const uint32_t e = blockIdx.x * 256u + threadIdx.x;
     if (e >= pieces) return;
-    const uint32_t r = e / k8, first = r * row_step + (e - r * k8) * 8u * col_step + seed;
-    float v[8];
+    const uint32_t lane = e & 63u, unit = e >> 6, rb = unit / ksteps, ks = unit - rb * ksteps, r = rb * 32u + (lane & 31u), c = ks * 16u + (lane >> 5) * 8u;
+    i32x4 h = {0, 0, 0, 0};
+    if (r < rows && c < cols) {   // cols is a multiple of 8
+        const uint32_t first = r * row_step + c * col_step + seed;
+        float v[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = (float)(int32_t)sq5_tail(first + (uint32_t)j * col_step) * 4.656612873077392578125e-10f;
-    i32x4 h;
+        for (int j = 0; j < 8; ++j) v[j] = (float)(int32_t)sq5_tail(first + (uint32_t)j * col_step) * 4.656612873077392578125e-10f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) h[j] = (int)f32x2_to_bf16x2(v[2 * j], v[2 * j + 1]);
+        for (int j = 0; j < 4; ++j) h[j] = (int)f32x2_to_bf16x2(v[2 * j], v[2 * j + 1]);
+    }
     *reinterpret_cast<i32x4 *>(out + (int64_t)e * 8) = h;
 }
-// rows x cols values, cols a multiple of 8, fewer than 2^29
-static int launch_noise_rows(void *out, int64_t rows, int64_t cols, uint32_t row_step, uint32_t col_step, uint32_t seed, hipStream_t s)
+// rows rounded up to 32, columns to 64
+static int64_t noise_frag_bytes(int64_t rows, int64_t cols) { return cdiv(rows, 32) * 32 * cdiv(cols, 64) * 64 * (int64_t)sizeof(bf16_t); }
+static int launch_noise_frag(void *out, int64_t rows, int64_t cols, uint32_t row_step, uint32_t col_step, uint32_t seed, hipStream_t s)
 {
-    const uint32_t pieces = (uint32_t)(rows * cols / 8);
-    noise_rows_bf16_kernel<<<(unsigned)cdiv(pieces, 256), 256, 0, s>>>(static_cast<bf16_t *>(out), pieces, (uint32_t)(cols / 8), row_step, col_step, seed);
-    return check_launch("noise_rows_bf16_kernel");
+    const uint32_t pieces = (uint32_t)(noise_frag_bytes(rows, cols) / 16);
+    noise_frag_bf16_kernel<<<(unsigned)cdiv(pieces, 256), 256, 0, s>>>(static_cast<bf16_t *>(out), pieces, (uint32_t)(cdiv(cols, 64) * 4), (uint32_t)rows,
+                                                                       (uint32_t)cols, row_step, col_step, seed);
+    return check_launch("noise_frag_bf16_kernel");
 }
 
 // Scratch for N^T where dx = t . N takes it from memory; 0: where it does not.
 int64_t dx_big_table_bytes(const rdb_linear_desc *d, int num_cus)
 {
     const ProjLayout L = proj_layout(d);
-    if (!L.ok || L.fits_regs || d->in_f * d->k >= (1ll << 29) || !enough_tiles(cdiv(d->in_f, BG) * cdiv(d->tokens, BG), num_cus)) return 0;
-    return (d->in_f * d->k * (int64_t)sizeof(bf16_t) + 255) / 256 * 256;
+    if (!L.ok || L.fits_regs || noise_frag_bytes(d->in_f, d->k) >= (1ll << 30) || !enough_tiles(cdiv(d->in_f, BG) * cdiv(d->tokens, BG), num_cus)) return 0;
+    return noise_frag_bytes(d->in_f, d->k);
 }
 
 // dx = t . N with t [tokens x k] row-major and room for N^T at `table`
@@ -502,7 +653,7 @@ int linear_tn_big(void *dx, int64_t lddx, const void *t, void *table, const rdb_
 {
     if (!dx_big_table_bytes(d, num_cus) || lddx % 8 || d->tokens * lddx >= (1ll << 29) || !big_aligned16(dx) || !big_aligned16(t) || !big_aligned16(table))
         return RDB_E_UNSUPPORTED;
-    if (int rc = launch_noise_rows(table, d->in_f, d->k, PN1, SQ5_N1, d->seed, s)) return rc;   // N^T[i, m] = noise(PRIME * i + m)
+    if (int rc = launch_noise_frag(table, d->in_f, d->k, PN1, SQ5_N1, d->seed, s)) return rc;   // N^T[i, m] = noise(PRIME * i + m)
     BigYParams p = {};
     p.zf = static_cast<const bf16_t *>(t);
     p.coef = static_cast<const bf16_t *>(table);
@@ -515,7 +666,7 @@ int linear_tn_big(void *dx, int64_t lddx, const void *t, void *table, const rdb_
     p.tiles_o = (int)cdiv(d->in_f, BG);
     p.tiles_t = (int)cdiv(d->tokens, BG);
     typedef OperandTile<BG, 64, K_CONT> TA;
-    return launch_big(big_y_kernel<false, false>, p, p.tiles_o * p.tiles_t, num_cus, big_smem<BG, BG, TA, TA>(), s, "big_y_kernel (dx = t . N)");
+    return launch_big(big_y_kernel<false, false>, p, p.tiles_o * p.tiles_t, num_cus, big_smem<BG, BG, FragTile<BG, 64>, TA>(), s, "big_y_kernel (dx = t . N)");
 }
 
 // state <- z (and C transposed, with coef), N in `room` (room_bytes of it; the rows of the forward product to come will do)
@@ -524,11 +675,11 @@ int linear_z_big(void *state, const void *x, int64_t ldx, const void *coef, void
 {
     const ProjLayout L = proj_layout(d);
     const int64_t tiles = cdiv(d->k, BG) * cdiv(d->tokens, BZ_TOK);
-    if (!L.ok || L.fits_regs || !enough_tiles(tiles, num_cus) || d->in_f * d->k >= (1ll << 29) || !room || room_bytes < d->in_f * d->k * 2)
+    if (!L.ok || L.fits_regs || !enough_tiles(tiles, num_cus) || noise_frag_bytes(d->k, d->in_f) >= (1ll << 30) || !room || room_bytes < noise_frag_bytes(d->k, d->in_f))
         return RDB_E_UNSUPPORTED;
     if (ldx % 8 || d->tokens * ldx >= (1ll << 29) || !big_aligned16(x) || !big_aligned16(state) || !big_aligned16(coef) || !big_aligned16(room))
         return RDB_E_UNSUPPORTED;
-    if (int rc = launch_noise_rows(room, d->k, d->in_f, SQ5_N1, PN1, d->seed, s)) return rc;   // N[m, i] = noise(PRIME * i + m)
+    if (int rc = launch_noise_frag(room, d->k, d->in_f, SQ5_N1, PN1, d->seed, s)) return rc;   // N[m, i] = noise(PRIME * i + m)
     char *st = static_cast<char *>(state);
     BigZParams p;
     p.noise = static_cast<const bf16_t *>(room);
@@ -550,13 +701,53 @@ int linear_z_big(void *state, const void *x, int64_t ldx, const void *coef, void
     p.tiles_m = (int)cdiv(d->k, BG);
     p.tiles_t = (int)cdiv(d->tokens, BZ_TOK);
     p.tile_blocks = xcd_grid_size((int)tiles);
-    const size_t smem = big_smem<BG, BZ_TOK, OperandTile<BG, 64, K_CONT>, OperandTile<BZ_TOK, 64, K_CONT>>();
+    const size_t smem = big_smem<BG, BZ_TOK, FragTile<BG, 64>, OperandTile<BZ_TOK, 64, K_CONT>>();
     if (int rl = reserve_lds(reinterpret_cast<const void *>(big_z_kernel), smem, "big_z_kernel")) return rl;
     // the transposing blocks: the compute units that the tiles leave free, or as many as there are
     int c_blocks = coef ? num_cus - p.tile_blocks : 0;
     if (coef && c_blocks < num_cus / 4) c_blocks = num_cus;
     big_z_kernel<<<p.tile_blocks + c_blocks, 256, smem, s>>>(p);
     return check_launch("big_z_kernel");
+}
+
+// Scratch for R where the random bias's share of [tokens x cols] takes it from memory; 0: where it does not (too few tiles, or more
+// than the activations of the pass take).
+int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus)
+{
+    const int64_t n = d->in_f * d->out_f, bytes = noise_frag_bytes(cols, cols == d->in_f ? d->out_f : d->in_f);
+    if (d->act_dtype != RDB_BF16 || d->in_f % 8 || d->out_f % 8 || d->in_f < 8 || d->out_f < 8 || bytes >= (1ll << 30) ||
+        n > d->tokens * (d->in_f + d->out_f) || !enough_tiles(cdiv(cols, BG) * cdiv(d->tokens, BR_TOK), num_cus))
+        return 0;
+    return bytes;
+}
+
+// dst[t, a] += s * sum_c src[t, c] * noise1d(a * sR + c * sK); with `other` also one sum per tile to dot_part, *tiles of them.  The caller
+// has checked alignments and extents.
+int linear_rbias_big(void *dst, int64_t ld_dst, int64_t cols, const void *src, int64_t ld_src, int64_t contraction, uint32_t sR, uint32_t sK,
+                     const void *scale, const rdb_linear_desc *d, void *table, const void *other, int64_t ld_other, float *dot_part, int *tiles,
+                     int num_cus, hipStream_t s)
+{
+    if (int rc = launch_noise_frag(table, cols, contraction, sR * SQ5_N1, sK * SQ5_N1, d->seed, s)) return rc;
+    BigRBiasParams p;
+    p.noise = static_cast<const bf16_t *>(table);
+    p.src = static_cast<const bf16_t *>(src);
+    p.dst = static_cast<bf16_t *>(dst);
+    p.scale = static_cast<const bf16_t *>(scale);
+    p.other = static_cast<const bf16_t *>(other);
+    p.dot_part = dot_part;
+    p.ld_src = ld_src;
+    p.ld_dst = ld_dst;
+    p.ld_other = ld_other;
+    p.tokens = (int)d->tokens;
+    p.cols = (int)cols;
+    p.contraction = (int)contraction;
+    p.tiles_a = (int)cdiv(cols, BG);
+    p.tiles_t = (int)cdiv(d->tokens, BR_TOK);
+    *tiles = p.tiles_a * p.tiles_t;
+    constexpr size_t stages = big_smem<BG, BR_TOK, FragTile<BG, 64>, OperandTile<BR_TOK, 64, K_CONT>>();
+    static_assert((size_t)4 * 32 * (BG / 2 + 4) * sizeof(float) <= stages, "the epilogue's patches fit the pipeline's LDS");
+    if (other) return launch_big(big_rbias_kernel<true>, p, *tiles, num_cus, stages, s, "big_rbias_kernel<dot>");
+    return launch_big(big_rbias_kernel<false>, p, *tiles, num_cus, stages, s, "big_rbias_kernel");
 }
 
 // First launch of the backward pass: t (row-major, for the t . N kernel of the tile engine) and dC.  `dc`: where the

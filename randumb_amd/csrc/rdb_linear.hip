@@ -349,11 +349,12 @@ int linear_bwd_big(void *t, void *dc, bool dc_bf16, const void *dy, int64_t lddy
 int64_t dx_big_table_bytes(const rdb_linear_desc *d, int num_cus);
 
 // rdb_rbias.hip
-int linear_dx_rbias_add(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s);
-int linear_fwd_rbias_add(void *y, int64_t ldy, const void *x, int64_t ldx, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s);
+int linear_dx_rbias_add(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table = nullptr, int64_t table_bytes = 0);
+int linear_fwd_rbias_add(void *y, int64_t ldy, const void *x, int64_t ldx, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table = nullptr, int64_t table_bytes = 0);
 int64_t linear_dx_rbias_dot_floats(const rdb_linear_desc *d);
 int linear_dx_rbias_add_dscale(void *dx, int64_t lddx, float *dscale, float *dot_part, const void *dy, int64_t lddy, const void *x, int64_t ldx,
-                               const void *scale_bias, const rdb_linear_desc *d, hipStream_t s);
+                               const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table = nullptr, int64_t table_bytes = 0);
+int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);   // rdb_big.hip
 
 // rdb_vecsplit.hip
 int64_t linear_vecsplit_workspace(int op, const rdb_linear_desc *d);
@@ -439,6 +440,7 @@ extern "C" int64_t rdb_linear_workspace_bytes(int op, const rdb_linear_desc *d)
     return need;
 }
 
+static int64_t rbias_dot_room(const rdb_linear_desc *d) { return (linear_dx_rbias_dot_floats(d) * 4 + 255) / 256 * 256; }
 static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d)
 {
     if (d->algo == RDB_ALGO_TILE || d->algo == RDB_ALGO_STRIP) return 0;
@@ -469,8 +471,13 @@ static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d)
         const int64_t t = linear_dx_factored_workspace(d);
         return t > 0 ? (t + 255) / 256 * 256 + linear_dx_rbias_dot_floats(d) * 4 : 0;
     }
-    if (op == RDB_OP_LINEAR_RBIAS_BWD)   // one float per tile of the random-bias product (the gradient of the scale)
-        return (d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16 && d->in_f % 8 == 0 && d->out_f % 8 == 0) ? linear_dx_rbias_dot_floats(d) * 4 : 0;
+    if (op == RDB_OP_LINEAR_RBIAS_BWD) {   // one float per tile of the random-bias product (the gradient of the scale); behind them R, never required
+        if (d->act_dtype != RDB_BF16 || d->coef_dtype != RDB_BF16 || d->in_f % 8 || d->out_f % 8) return 0;
+        const int64_t table = rbias_big_table_bytes(d, d->in_f, num_compute_units());
+        return table > 0 ? rbias_dot_room(d) + table : linear_dx_rbias_dot_floats(d) * 4;
+    }
+    if (op == RDB_OP_LINEAR_RBIAS_FWD)
+        return d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16 ? rbias_big_table_bytes(d, d->out_f, num_compute_units()) : 0;
     if (op == RDB_OP_LINEAR_BWD_PROJECTED || op == RDB_OP_LINEAR_BWD_PROJECTED_TO) {
         const int64_t base = bwd_projected_workspace(d, op == RDB_OP_LINEAR_BWD_PROJECTED_TO), table = base > 0 ? bwd_projected_table(d) : 0;
         return table > 0 ? (base + 255) / 256 * 256 + table : base;   // what lies behind `base` is never required
@@ -702,12 +709,18 @@ static int rbias_request_ok(const char *who, const rdb_linear_desc *d)
 
 extern "C" int rdb_linear_rbias_fwd(void *y, int64_t ldy, const void *x, int64_t ldx, const void *scale_bias, const rdb_linear_desc *d, void *stream)
 {
+    return rdb_linear_rbias_fwd_ws(y, ldy, x, ldx, scale_bias, d, nullptr, 0, stream);
+}
+
+extern "C" int rdb_linear_rbias_fwd_ws(void *y, int64_t ldy, const void *x, int64_t ldx, const void *scale_bias, const rdb_linear_desc *d, void *workspace,
+                                       int64_t workspace_bytes, void *stream)
+{
     int rc = check_desc("rdb_linear_rbias_fwd", d);
     if (rc) return rc;
     if (!y || !x || !scale_bias) return set_error(RDB_E_NULL, "rdb_linear_rbias_fwd: y, x or scale_bias is NULL");
     if (ldy < d->out_f || ldx < d->in_f) return set_error(RDB_E_SHAPE, "rdb_linear_rbias_fwd: leading dimension smaller than the row");
     if ((rc = rbias_request_ok("rdb_linear_rbias_fwd", d))) return rc;
-    rc = linear_fwd_rbias_add(y, ldy, x, ldx, scale_bias, d, (hipStream_t)stream);
+    rc = linear_fwd_rbias_add(y, ldy, x, ldx, scale_bias, d, (hipStream_t)stream, workspace, workspace_bytes);
     if (rc == RDB_E_UNSUPPORTED)
         return set_error(RDB_E_UNSUPPORTED, "rdb_linear_rbias_fwd: needs 16-byte aligned rows (pointers and leading dimensions) and fewer than "
                                             "2^29 elements per matrix");
@@ -724,16 +737,19 @@ extern "C" int rdb_linear_rbias_bwd(void *dx, int64_t lddx, float *d_scale_bias,
     if ((rc = rbias_request_ok("rdb_linear_rbias_bwd", d))) return rc;
     const char *why = "rdb_linear_rbias_bwd: needs 16-byte aligned rows (pointers and leading dimensions) and fewer than 2^29 elements per matrix";
     hipStream_t s = (hipStream_t)stream;
+    // R behind the room for the tiles' sums, whether they are wanted or not
+    const int64_t dots = rbias_dot_room(d), room = workspace ? std::max<int64_t>(0, workspace_bytes - dots) : 0;
+    void *const table = room > 0 ? static_cast<char *>(workspace) + dots : nullptr;
     if (!d_scale_bias) {
-        rc = linear_dx_rbias_add(dx, lddx, dy, lddy, scale_bias, d, s);
+        rc = linear_dx_rbias_add(dx, lddx, dy, lddy, scale_bias, d, s, table, room);
         return rc == RDB_E_UNSUPPORTED ? set_error(RDB_E_UNSUPPORTED, "%s", why) : rc;
     }
     if (!x) return set_error(RDB_E_NULL, "rdb_linear_rbias_bwd: the gradient of the scale needs x");
     if (ldx < d->in_f) return set_error(RDB_E_SHAPE, "rdb_linear_rbias_bwd: leading dimension smaller than the row");
-    const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_BWD, d);
+    const int64_t need = linear_dx_rbias_dot_floats(d) * 4;
     if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 3))
         return set_error(RDB_E_WORKSPACE, "rdb_linear_rbias_bwd: the gradient of the scale needs a workspace of %lld bytes", (long long)need);
-    rc = linear_dx_rbias_add_dscale(dx, lddx, d_scale_bias, static_cast<float *>(workspace), dy, lddy, x, ldx, scale_bias, d, s);
+    rc = linear_dx_rbias_add_dscale(dx, lddx, d_scale_bias, static_cast<float *>(workspace), dy, lddy, x, ldx, scale_bias, d, s, table, room);
     return rc == RDB_E_UNSUPPORTED ? set_error(RDB_E_UNSUPPORTED, "%s", why) : rc;
 }
 

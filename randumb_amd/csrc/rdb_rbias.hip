@@ -8,13 +8,19 @@
 //     y[t, o]  += s * sum_i x[t, i]  * R[o, i]        (forward, where no kernel that forms W strips fits)
 // on the tile engine with R as a hashed operand: a tile of 64 features x 256 tokens, R hashed once per block and
 // stage straight into the pipeline's registers (as 2^31 * noise in bf16, the scale folded into the epilogue), two blocks
-// per compute unit so that one block's hashing runs under the other's matrix work.  R never exists in memory.
+// per compute unit so that one block's hashing runs under the other's matrix work.  R never exists in memory; with scratch for it
+// that is no larger than the activations, and tiles enough, the product runs on the 256-wide tiles of rdb_big.hip instead.
 #include "rdb_gemm.hpp"
 #include "rdb_tile.hpp"
 
 namespace rdb {
 
 int num_compute_units();   // of the current device (rdb_error.hip)
+// rdb_big.hip
+int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);
+int linear_rbias_big(void *dst, int64_t ld_dst, int64_t cols, const void *src, int64_t ld_src, int64_t contraction, uint32_t sR, uint32_t sK,
+                     const void *scale, const rdb_linear_desc *d, void *table, const void *other, int64_t ld_other, float *dot_part, int *tiles,
+                     int num_cus, hipStream_t s);
 
 constexpr int RB_BI = 64, RB_BT = 256, RB_BK = 64;
 
@@ -367,10 +373,14 @@ __global__ __launch_bounds__(256) void rbias_sum_kernel(float *__restrict__ out,
     if (threadIdx.x == 0) out[0] = sh[0];
 }
 
-// other / dot_part / dscale: NULL, or the matrix the product is reduced against, room for one float per tile, and where the sum goes
+// floats of scratch for the tiles' shares of the scale's gradient
+int64_t linear_dx_rbias_dot_floats(const rdb_linear_desc *d) { return cdiv(d->in_f, RB_BI) * cdiv(d->tokens, RB_BT); }
+
+// other / dot_part / dscale: NULL, or the matrix the product is reduced against, room for one float per tile, and where the sum goes;
+// table: NULL, or scratch of table_bytes for R
 static int rbias_add(void *dst, int64_t ld_dst, int64_t cols, const void *src, int64_t ld_src, int64_t contraction, uint32_t sR, uint32_t sK,
                      const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, const void *other = nullptr, int64_t ld_other = 0,
-                     float *dot_part = nullptr, float *dscale = nullptr)
+                     float *dot_part = nullptr, float *dscale = nullptr, void *table = nullptr, int64_t table_bytes = 0)
 {
     if (d->act_dtype != RDB_BF16 || d->coef_dtype != RDB_BF16 || d->coef_rows == 0 || !scale_bias) return RDB_E_UNSUPPORTED;
     if (d->in_f % 8 || d->out_f % 8 || d->tokens < 1 || d->in_f < 1 || d->out_f < 1) return RDB_E_UNSUPPORTED;
@@ -394,6 +404,16 @@ static int rbias_add(void *dst, int64_t ld_dst, int64_t cols, const void *src, i
     p.ld_other = ld_other;
     p.dot_part = dot_part;
     if (other && (ld_other % 8 || ((uintptr_t)other & 15) || d->tokens * ld_other >= (1ll << 29) || !dot_part || !dscale)) return RDB_E_UNSUPPORTED;
+    const int64_t need = table ? rbias_big_table_bytes(d, cols, num_compute_units()) : 0;
+    if (need > 0 && table_bytes >= need && !((uintptr_t)table & 15) && (!other || cdiv(cols, 256) * cdiv(d->tokens, 128) <= linear_dx_rbias_dot_floats(d))) {
+        int tiles = 0;
+        if (int rc = linear_rbias_big(dst, ld_dst, cols, src, ld_src, contraction, sR, sK, scale_bias, d, table, other, ld_other, dot_part, &tiles,
+                                      num_compute_units(), s))
+            return rc;
+        if (!other) return RDB_OK;
+        rbias_sum_kernel<<<1, 256, 0, s>>>(dscale, dot_part, tiles);
+        return check_launch("rbias_sum_kernel");
+    }
     // tiles of 512 tokens when they give at least every other compute unit a block (half the hashing per product: measured
     // ahead from there on; 8192 tokens x 768 features, contraction 3072: 83 -> 67 us), tiles of 256 tokens otherwise
     const int wide_items = (int)(cdiv(cols, RW_BI) * cdiv(d->tokens, RW_BT));
@@ -422,27 +442,26 @@ static int rbias_add(void *dst, int64_t ld_dst, int64_t cols, const void *src, i
     return check_launch("rbias_sum_kernel");
 }
 
-// floats of scratch for the tiles' shares of the scale's gradient
-int64_t linear_dx_rbias_dot_floats(const rdb_linear_desc *d) { return cdiv(d->in_f, RB_BI) * cdiv(d->tokens, RB_BT); }
-
 // dx += s * dy . R and d s = <dy . R, x> in one pass over dy . R
 int linear_dx_rbias_add_dscale(void *dx, int64_t lddx, float *dscale, float *dot_part, const void *dy, int64_t lddy, const void *x, int64_t ldx,
-                               const void *scale_bias, const rdb_linear_desc *d, hipStream_t s)
+                               const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table, int64_t table_bytes)
 {
-    return rbias_add(dx, lddx, d->in_f, dy, lddy, d->out_f, 1u, (uint32_t)d->in_f, scale_bias, d, s, x, ldx, dot_part, dscale);
+    return rbias_add(dx, lddx, d->in_f, dy, lddy, d->out_f, 1u, (uint32_t)d->in_f, scale_bias, d, s, x, ldx, dot_part, dscale, table, table_bytes);
 }
 
 // dx += s * dy . R on the launch stream, after the kernels that wrote dx.  Returns RDB_E_UNSUPPORTED (without setting an
 // error) when the request does not fit.
-int linear_dx_rbias_add(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s)
+int linear_dx_rbias_add(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table,
+                        int64_t table_bytes)
 {
-    return rbias_add(dx, lddx, d->in_f, dy, lddy, d->out_f, 1u, (uint32_t)d->in_f, scale_bias, d, s);
+    return rbias_add(dx, lddx, d->in_f, dy, lddy, d->out_f, 1u, (uint32_t)d->in_f, scale_bias, d, s, nullptr, 0, nullptr, nullptr, table, table_bytes);
 }
 
 // y += s * x . R^T on the launch stream, after the kernels that wrote y; same conditions.
-int linear_fwd_rbias_add(void *y, int64_t ldy, const void *x, int64_t ldx, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s)
+int linear_fwd_rbias_add(void *y, int64_t ldy, const void *x, int64_t ldx, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table,
+                         int64_t table_bytes)
 {
-    return rbias_add(y, ldy, d->out_f, x, ldx, d->in_f, (uint32_t)d->in_f, 1u, scale_bias, d, s);
+    return rbias_add(y, ldy, d->out_f, x, ldx, d->in_f, (uint32_t)d->in_f, 1u, scale_bias, d, s, nullptr, 0, nullptr, nullptr, table, table_bytes);
 }
 
 }  // namespace rdb

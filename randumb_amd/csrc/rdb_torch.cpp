@@ -350,7 +350,9 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         if (scale_bias) {
             const Tensor sb = native(*scale_bias).to(at::kBFloat16);
             const rdb_linear_desc r = rbias_desc(x, l);
-            check(rdb_linear_rbias_fwd(y.data_ptr(), l.out_f, x.data_ptr(), x.stride(0), sb.data_ptr(), &r, s), "rdb_linear_rbias_fwd");
+            const int64_t room = rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_FWD, &r);
+            const Tensor ws = bytes(room, x);
+            check(rdb_linear_rbias_fwd_ws(y.data_ptr(), l.out_f, x.data_ptr(), x.stride(0), sb.data_ptr(), &r, ptr(ws), room, s), "rdb_linear_rbias_fwd");
         }
         tick(x);
         ctx->save_for_backward({state, coefs, scale_bias.value_or(Tensor()), scale_bias ? x0 : Tensor()});
@@ -399,16 +401,16 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         if (has_sb && dx.defined()) {
             const Tensor x = act(saved[3]), sb = native(scale_bias).to(at::kBFloat16);
             const rdb_linear_desc r = rbias_desc(dy, l);
+            const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_BWD, &r);
+            const Tensor ws = bytes(need, dy);
             if (want_sb) {
-                const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_BWD, &r);
-                const Tensor ws = bytes(need, dy);
                 dsb = at::empty({1}, dy.options().dtype(at::kFloat));
                 check(rdb_linear_rbias_bwd(dx.data_ptr(), l.in_f, dsb.data_ptr<float>(), dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), sb.data_ptr(),
                                            &r, ptr(ws), need, s),
                       "rdb_linear_rbias_bwd");
                 dsb = dsb.to(scale_bias.scalar_type());
             } else {
-                check(rdb_linear_rbias_bwd(dx.data_ptr(), l.in_f, nullptr, dy.data_ptr(), dy.stride(0), nullptr, 0, sb.data_ptr(), &r, nullptr, 0, s),
+                check(rdb_linear_rbias_bwd(dx.data_ptr(), l.in_f, nullptr, dy.data_ptr(), dy.stride(0), nullptr, 0, sb.data_ptr(), &r, ptr(ws), need, s),
                       "rdb_linear_rbias_bwd");
             }
         }

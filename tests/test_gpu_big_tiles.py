@@ -251,7 +251,7 @@ def test_backward_with_the_noise_from_memory(T, in_f, out_f, k):
     try:
         y, state = hip.linear_project_fwd(x, c, 5)
         full = lib.rdb_linear_workspace_bytes(4, ref)
-        table = -(-in_f * k * 2 // 256) * 256
+        table = -(-in_f // 32) * 32 * -(-k // 64) * 64 * 2
         results = []
         for size, dtype in ((full, torch.bfloat16), (full - table, torch.bfloat16), (full, torch.float32)):
             dx, dc = torch.empty_like(x), torch.empty(out_f, k, dtype=dtype, device="cuda")
@@ -287,3 +287,41 @@ def test_projection_with_the_noise_from_memory(hip, T, in_f, out_f, k):
     finally:
         hip.set_big_tiles(before)
     assert torch.equal(y, want[0]) and torch.equal(dx, want[1]) and torch.equal(dx, dx_alone) and torch.equal(dc, dc_alone)
+
+
+@pytest.mark.parametrize("T,in_f,out_f", [(300, 264, 520), (129, 8, 1032), (513, 1000, 72), (128, 64, 64), (2056, 520, 776)])
+def test_random_bias_from_memory(T, in_f, out_f):
+    """The random bias's share on 256-wide tiles against the kernels that hash it: the same bits in y and dx (the same products in the same
+    order); the scale's gradient adds the same terms up in other groups (fp32)."""
+    import ctypes
+
+    from randumb_amd import _lib, hip
+
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(T)
+    x, dy = torch.randn(T, in_f, generator=g).bfloat16().cuda(), torch.randn(T, out_f, generator=g).bfloat16().cuda()
+    y0, dx0 = torch.randn(T, out_f, generator=g).bfloat16().cuda(), torch.randn(T, in_f, generator=g).bfloat16().cuda()
+    s = torch.tensor([0.375]).bfloat16().cuda()
+    ref = ctypes.byref(hip._rbias_desc(T, in_f, out_f, 9))
+    stream = torch.cuda.current_stream().cuda_stream
+    old = lib.rdb_set_big_tiles(2)
+    try:
+        dots = -(-in_f // 64) * -(-T // 256) * 4
+        out = []
+        for table in (True, False):
+            fwd, bwd = [lib.rdb_linear_workspace_bytes(op, ref) if table else n for op, n in ((8, 0), (6, dots))]
+            if table:
+                assert fwd >= in_f * out_f * 2 and bwd >= dots + in_f * out_f * 2
+            y, dx, dx_only, ds = y0.clone(), dx0.clone(), dx0.clone(), torch.empty(1, device="cuda")
+            ws = torch.empty(max(fwd, bwd, 256), dtype=torch.uint8, device="cuda")
+            assert lib.rdb_linear_rbias_fwd_ws(y.data_ptr(), out_f, x.data_ptr(), in_f, s.data_ptr(), ref, ws.data_ptr(), fwd, stream) == 0
+            assert lib.rdb_linear_rbias_bwd(dx.data_ptr(), in_f, ds.data_ptr(), dy.data_ptr(), out_f, x.data_ptr(), in_f, s.data_ptr(), ref, ws.data_ptr(), bwd,
+                                            stream) == 0
+            assert lib.rdb_linear_rbias_bwd(dx_only.data_ptr(), in_f, None, dy.data_ptr(), out_f, None, 0, s.data_ptr(), ref, ws.data_ptr(), bwd, stream) == 0
+            assert torch.equal(dx, dx_only)
+            out.append((y, dx, float(ds)))
+    finally:
+        lib.rdb_set_big_tiles(old)
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    # the sum of T * in_f terms of mean square out_f / 3: fp32 roundings of it, in two orders
+    assert abs(out[0][2] - out[1][2]) < 1e-5 * (T * in_f * out_f / 3) ** 0.5

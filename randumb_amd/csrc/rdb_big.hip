@@ -4,6 +4,7 @@
 //   big_bwd_kernel  t[tok, m]  = sum_o dy[tok, o] * C[o, m]                       256 (m) x 128 (tok) tiles, and in the same launch
 //                   dC[o, m]   = sum_tok dy[tok, o] * z[tok, m]                   256 (o) x 256 (m) tiles over all tokens
 //   big_z_kernel    z[tok, m]  = sum_i x[tok, i] * N[m, i]                        256 (m) x 128 (tok) tiles, N from memory
+//   big_yr_kernel   y[tok, o]  = z . C^T + s * x . R^T (any k)                    256 (o) x 128 (tok) tiles, R from memory
 //   big_rbias_kernel  y += s * x . R^T,  dx += s * dy . R (any k)                 256 (features) x 128 (tok) tiles, R from memory
 //   big_y_kernel    dx[tok, i] = sum_m t[tok, m] * N[m, i]                        256 (i) x 256 (tok) tiles, N from memory
 // z, z^T and C^T come from the projection state in fragment order (rdb_direct.hpp: ProjLayout).  One persistent block per
@@ -554,6 +555,78 @@ template <bool DOT> __global__ __launch_bounds__(256, 1) void big_rbias_kernel(B
     }
 }
 
+// ----------------------------------------------------------------------------------------------- y = z . C^T + s * x . R^T (+ bias)
+// A forward pass with the fused random bias in one product: the tile's accumulators contract in_f (x with R), are scaled, and go on with
+// k (z with C), so that y is written once, rounded once, and never read back (8192 tokens x 768 -> 3072, k = 256: y = z . C^T beside the
+// projection and y += s x . R^T: 98 us; z, R and this: 84).  Tiles of 256 output features x 128 tokens, one persistent block a compute unit.
+struct BigYRParams {
+    const bf16_t *noise;   // R [out_f x in_f] in fragment order
+    const bf16_t *x;
+    const bf16_t *zf;      // fragment order, rows = tokens
+    const bf16_t *coef;    // [out_f x k]
+    const bf16_t *scale;   // one value
+    const bf16_t *bias;
+    bf16_t *y;
+    int64_t ldx, ldy;
+    int tokens, in_f, out_f, k, tiles_o, tiles_t;
+};
+
+template <bool BIAS> __global__ __launch_bounds__(256, 1) void big_yr_kernel(BigYRParams p)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
+    typedef FragOperand<BG, 64> PR;                  // R: rows = output features
+    typedef GlobalOperand<BR_TOK, 64, K_CONT> PX;    // x: rows = tokens
+    typedef GlobalOperand<BG, 64, K_CONT> PC;        // C: rows = output features
+    typedef FragOperand<BR_TOK, 64> PZ;              // z: rows = tokens
+    constexpr int MI = BG / 64, NI = BR_TOK / 64;
+    const int total = p.tiles_o * p.tiles_t, vtotal = (total + 7) / 8 * 8, nblk = gridDim.x;
+    int rd = 0;
+    auto next = [&]() {
+        for (; rd * nblk + (int)blockIdx.x < vtotal; ++rd) {
+            const int w = xcd_work_item(rd * nblk + (int)blockIdx.x, total);
+            if (w < total) { ++rd; return w; }
+        }
+        return -1;
+    };
+    PR pr;
+    PX px;
+    BigRegs<PR, PX> regs;
+    auto request = [&](int w) {   // output tile fastest: neighbours share the tokens
+        frag_rows(pr, p.noise, p.out_f, p.in_f, (w % p.tiles_o) * BG);
+        px = PX{p.x, p.ldx, (w / p.tiles_o) * BR_TOK, p.tokens, p.in_f, (int64_t)(p.tokens - 1) * p.ldx + p.in_f};
+        big_prefetch(regs, pr, px, 0);
+    };
+    int w = next();
+    if (w < 0) return;
+    request(w);
+    const float sval = bf16_to_f32(*p.scale);
+    while (true) {
+        const int o0 = (w % p.tiles_o) * BG, tok0 = (w / p.tiles_o) * BR_TOK;
+        PC pc = {p.coef, (int64_t)p.k, o0, p.out_f, p.k, (int64_t)p.out_f * p.k};
+        PZ pz;
+        frag_rows(pz, p.zf, p.tokens, p.k, tok0);
+        BigRegs<PC, PZ> regs2;
+        big_prefetch(regs2, pc, pz, 0);
+        f32x16 acc[MI][NI];
+        big_zero<BG, BR_TOK>(acc);
+        big_mainloop<BG, BR_TOK>(acc, lds, regs, pr, px, (p.in_f + 63) / 64);
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni) acc[mi][ni] *= sval;
+        big_mainloop<BG, BR_TOK>(acc, lds, regs2, pc, pz, (p.k + 63) / 64);
+        BigBias<BG> bias;
+        if (BIAS) big_load_bias<BG>(bias, p.bias, o0, p.out_f);
+        const int wn = next();
+        if (wn >= 0) request(wn);
+        __builtin_amdgcn_sched_barrier(0);
+        big_store_bf16<BG, BR_TOK, BIAS, true>(acc, lds, p.y, p.ldy, (int64_t)(p.tokens - 1) * p.ldy + p.out_f, o0, p.out_f, tok0, p.tokens, bias, opaque_tid());
+        if (wn < 0) break;
+        w = wn;
+    }
+}
+
 // ----------------------------------------------------------------------------------------------- host side
 static bool big_aligned16(const void *q) { return ((uintptr_t)q & 15) == 0; }
 
@@ -748,6 +821,38 @@ int linear_rbias_big(void *dst, int64_t ld_dst, int64_t cols, const void *src, i
     static_assert((size_t)4 * 32 * (BG / 2 + 4) * sizeof(float) <= stages, "the epilogue's patches fit the pipeline's LDS");
     if (other) return launch_big(big_rbias_kernel<true>, p, *tiles, num_cus, stages, s, "big_rbias_kernel<dot>");
     return launch_big(big_rbias_kernel<false>, p, *tiles, num_cus, stages, s, "big_rbias_kernel");
+}
+
+// y = z . C^T + s * x . R^T (+ bias) from the state, R in `table` (rbias_big_table_bytes of out_f columns)
+int linear_fwd_rbias_big(void *y, int64_t ldy, const void *x, int64_t ldx, const void *state, const void *coef, const void *scale, const void *bias,
+                         const rdb_linear_desc *d, void *table, int num_cus, hipStream_t s)
+{
+    const ProjLayout L = proj_layout(d);
+    if (!L.ok || d->coef_dtype != RDB_BF16 || ldx % 8 || ldy % 8 || d->tokens * ldx >= (1ll << 29) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
+    if (!big_aligned16(y) || !big_aligned16(x) || !big_aligned16(state) || !big_aligned16(coef) || !big_aligned16(table) || ((uintptr_t)bias & 7))
+        return RDB_E_UNSUPPORTED;
+    if (int rc = launch_noise_frag(table, d->out_f, d->in_f, (uint32_t)d->in_f * SQ5_N1, SQ5_N1, d->seed, s)) return rc;   // R[o, i] = noise1d(o * in_f + i)
+    BigYRParams p;
+    p.noise = static_cast<const bf16_t *>(table);
+    p.x = static_cast<const bf16_t *>(x);
+    p.zf = reinterpret_cast<const bf16_t *>(static_cast<const char *>(state) + L.zf_off);
+    p.coef = static_cast<const bf16_t *>(coef);
+    p.scale = static_cast<const bf16_t *>(scale);
+    p.bias = static_cast<const bf16_t *>(bias);
+    p.y = static_cast<bf16_t *>(y);
+    p.ldx = ldx;
+    p.ldy = ldy;
+    p.tokens = (int)d->tokens;
+    p.in_f = (int)d->in_f;
+    p.out_f = (int)d->out_f;
+    p.k = (int)d->k;
+    p.tiles_o = (int)cdiv(d->out_f, BG);
+    p.tiles_t = (int)cdiv(d->tokens, BR_TOK);
+    typedef OperandTile<BG, 64, K_CONT> TC;
+    typedef OperandTile<BR_TOK, 64, K_CONT> TX;
+    constexpr size_t one = big_smem<BG, BR_TOK, FragTile<BG, 64>, TX>(), two = big_smem<BG, BR_TOK, TC, FragTile<BR_TOK, 64>>(), smem = one > two ? one : two;
+    if (bias) return launch_big(big_yr_kernel<true>, p, p.tiles_o * p.tiles_t, num_cus, smem, s, "big_yr_kernel<bias>");
+    return launch_big(big_yr_kernel<false>, p, p.tiles_o * p.tiles_t, num_cus, smem, s, "big_yr_kernel");
 }
 
 // First launch of the backward pass: t (row-major, for the t . N kernel of the tile engine) and dC.  `dc`: where the

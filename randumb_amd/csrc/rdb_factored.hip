@@ -483,6 +483,18 @@ int linear_project(void *state, const void *x, int64_t ldx, const void *coef, co
     return launch_z(state, x, ldx, coef, nullptr, 0, d, s);
 }
 
+// The same ahead of a forward product: y's rows, contiguous and written last, hold N or sums on the way meanwhile.  With a contraction in
+// several ranges the 256-wide tiles' sums would differ from launch_z's (z_ranges).
+int linear_project_before(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, int num_cus,
+                          hipStream_t s)
+{
+    ZParams p;
+    if (!fill_z_params(p, state, x, ldx, coef, d)) return RDB_E_UNSUPPORTED;
+    const int64_t room = ldy == d->out_f && p.ranges == 1 ? d->tokens * d->out_f * (int64_t)sizeof(bf16_t) : 0;
+    const int rc = linear_z_big(state, x, ldx, coef, y, room, d, num_cus, s);
+    return rc != RDB_E_UNSUPPORTED ? rc : launch_z(state, x, ldx, coef, y, ldy, d, s);
+}
+
 // The forward product's parameters when the contraction of a token fits in registers (z in fragment order); returns the
 // number of work items, 0 when the request does not fit.
 static int fill_ys_params(StParams &q, void *y, int64_t ldy, const void *state, const void *coef, const void *bias, const rdb_linear_desc *d,
@@ -521,11 +533,7 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
         // check the second call's conditions before the first launch, so that a refusal leaves nothing half done
         if (d->coef_dtype != RDB_BF16 || ldy % 8 || !aligned16(y) || !aligned16(coef)) return RDB_E_UNSUPPORTED;
         if (((uintptr_t)bias & 7) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
-        // y's rows, contiguous and written last, hold N meanwhile; with a contraction in several ranges the sums differ (z_ranges)
-        const int64_t room = ldy == d->out_f && p.z.ranges == 1 ? d->tokens * d->out_f * (int64_t)sizeof(bf16_t) : 0;
-        int rc = linear_z_big(state, x, ldx, with_ct ? coef : nullptr, y, room, d, num_cus, s);
-        if (rc == RDB_E_UNSUPPORTED) rc = launch_z(state, x, ldx, with_ct ? coef : nullptr, y, ldy, d, s);
-        if (rc) return rc;
+        if (int rc = linear_project_before(state, x, ldx, with_ct ? coef : nullptr, y, ldy, d, num_cus, s)) return rc;
         return linear_fwd_projected(y, ldy, state, coef, bias, d, num_cus, s);
     }
     const ProjLayout L = proj_layout(d);

@@ -354,7 +354,12 @@ int linear_fwd_rbias_add(void *y, int64_t ldy, const void *x, int64_t ldx, const
 int64_t linear_dx_rbias_dot_floats(const rdb_linear_desc *d);
 int linear_dx_rbias_add_dscale(void *dx, int64_t lddx, float *dscale, float *dot_part, const void *dy, int64_t lddy, const void *x, int64_t ldx,
                                const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table = nullptr, int64_t table_bytes = 0);
-int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);   // rdb_big.hip
+// rdb_big.hip
+int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);
+int linear_project_before(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, int num_cus,
+                          hipStream_t s);   // rdb_factored.hip
+int linear_fwd_rbias_big(void *y, int64_t ldy, const void *x, int64_t ldx, const void *state, const void *coef, const void *scale, const void *bias,
+                         const rdb_linear_desc *d, void *table, int num_cus, hipStream_t s);
 
 // rdb_vecsplit.hip
 int64_t linear_vecsplit_workspace(int op, const rdb_linear_desc *d);
@@ -401,6 +406,7 @@ using namespace rdb;
 
 static int64_t bwd_projected_workspace(const rdb_linear_desc *d, bool force_partial);
 static int64_t bwd_projected_table(const rdb_linear_desc *d);
+static int64_t project_fwd_rbias_table(const rdb_linear_desc *d);
 
 // vector-coef coefficient gradient in two passes: dW = dy^T . x into the workspace (and the partial matrices of its token
 // ranges), then the contraction of rdb_materialize_bwd and, for the scale's gradient, of rdb_scale_bias_bwd, with their scratch
@@ -476,6 +482,7 @@ static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d)
         const int64_t table = rbias_big_table_bytes(d, d->in_f, num_compute_units());
         return table > 0 ? rbias_dot_room(d) + table : linear_dx_rbias_dot_floats(d) * 4;
     }
+    if (op == RDB_OP_LINEAR_PROJECT_FWD_RBIAS) return project_fwd_rbias_table(d);
     if (op == RDB_OP_LINEAR_RBIAS_FWD)
         return d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16 ? rbias_big_table_bytes(d, d->out_f, num_compute_units()) : 0;
     if (op == RDB_OP_LINEAR_BWD_PROJECTED || op == RDB_OP_LINEAR_BWD_PROJECTED_TO) {
@@ -1113,6 +1120,33 @@ extern "C" int rdb_linear_project_fwd(void *y, int64_t ldy, void *state, const v
         if (rc) return rc;
     }
     return RDB_OK;
+}
+
+static int64_t project_fwd_rbias_table(const rdb_linear_desc *d)
+{
+    if (d->act_dtype != RDB_BF16 || d->coef_dtype != RDB_BF16 || d->sO != d->in_f || d->sI != 1 || chunk_plan(d).nchunks != 1) return 0;
+    return rbias_big_table_bytes(d, d->out_f, num_compute_units());
+}
+
+extern "C" int rdb_linear_project_fwd_rbias(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, const void *scale_bias,
+                                            const void *bias, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
+{
+    const char *who = "rdb_linear_project_fwd_rbias";
+    if (int rc = check_desc(who, d)) return rc;
+    const int64_t need = project_fwd_rbias_table(d);
+    if (need <= 0) return set_error(RDB_E_UNSUPPORTED, "%s: a layer that has no such form (rdb_linear_workspace_bytes says 0)", who);
+    if (!y || !x || !state || !coef || !scale_bias) return set_error(RDB_E_NULL, "%s: y, x, state, coef or scale_bias is NULL", who);
+    if (ldy < d->out_f || ldx < d->in_f) return set_error(RDB_E_SHAPE, "%s: leading dimension smaller than the row", who);
+    if (!workspace || workspace_bytes < need) return set_error(RDB_E_WORKSPACE, "%s: needs a workspace of %lld bytes", who, (long long)need);
+    hipStream_t s = (hipStream_t)stream;
+    int rc = RDB_E_UNSUPPORTED;
+    if (ldx % 8 == 0 && ldy % 8 == 0 && aligned16(x) && aligned16(y) && aligned16(state) && aligned16(coef) && aligned16(workspace) && !((uintptr_t)bias & 7) &&
+        d->tokens * ldx < (1ll << 29) && d->tokens * ldy < (1ll << 29))
+        rc = linear_project_before(state, x, ldx, coef, y, ldy, d, num_compute_units(), s);
+    if (!rc) rc = linear_fwd_rbias_big(y, ldy, x, ldx, state, coef, scale_bias, bias, d, workspace, num_compute_units(), s);
+    if (rc == RDB_E_UNSUPPORTED)
+        return set_error(rc, "%s: 16-byte aligned pointers (bias: 8-byte), leading dimensions multiples of 8, fewer than 2^29 elements per matrix", who);
+    return rc;
 }
 
 extern "C" int rdb_linear_bwd_dcoef_projected(float *dcoef, const void *dy, int64_t lddy, const void *z, const rdb_linear_desc *d, void *stream)

@@ -346,8 +346,16 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         Tensor state = bytes(need, x), y = at::empty({x.size(0), l.out_f}, x.options());
         const Tensor b = pb.values(l.out_f, x.scalar_type());
         void *s = stream_of(x);
-        check(rdb_linear_project_fwd(y.data_ptr(), l.out_f, ptr(state), x.data_ptr(), x.stride(0), c.data_ptr(), ptr(b), &d, s), "rdb_linear_project_fwd");
-        if (scale_bias) {
+        const int64_t one_product = scale_bias ? rdb_linear_workspace_bytes(RDB_OP_LINEAR_PROJECT_FWD_RBIAS, &d) : 0;
+        if (one_product) {
+            const Tensor sb = native(*scale_bias).to(at::kBFloat16), ws = bytes(one_product, x);
+            check(rdb_linear_project_fwd_rbias(y.data_ptr(), l.out_f, ptr(state), x.data_ptr(), x.stride(0), c.data_ptr(), sb.data_ptr(), ptr(b), &d, ptr(ws),
+                                               one_product, s),
+                  "rdb_linear_project_fwd_rbias");
+        } else {
+            check(rdb_linear_project_fwd(y.data_ptr(), l.out_f, ptr(state), x.data_ptr(), x.stride(0), c.data_ptr(), ptr(b), &d, s), "rdb_linear_project_fwd");
+        }
+        if (scale_bias && !one_product) {
             const Tensor sb = native(*scale_bias).to(at::kBFloat16);
             const rdb_linear_desc r = rbias_desc(x, l);
             const int64_t room = rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_FWD, &r);

@@ -325,3 +325,44 @@ def test_random_bias_from_memory(T, in_f, out_f):
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
     # the sum of T * in_f terms of mean square out_f / 3: fp32 roundings of it, in two orders
     assert abs(out[0][2] - out[1][2]) < 1e-5 * (T * in_f * out_f / 3) ** 0.5
+
+
+@pytest.mark.parametrize("T,in_f,out_f,k,with_bias", [(300, 264, 520, 72, True), (129, 64, 1032, 264, False), (2056, 520, 776, 256, True), (513, 1000, 72, 328, False)])
+def test_forward_with_the_random_bias_in_one_product(T, in_f, out_f, k, with_bias):
+    """y = z . C^T + s * x . R^T + bias with one rounding: no further from float64 than the two products that round twice, the same state,
+    and the odd workspace refused."""
+    import ctypes
+
+    from randumb_amd import _lib, hip, ops
+
+    lib = _lib.load()
+    x, _, coef, bias = [t.cuda() for t in _inputs(T, in_f, out_f, k, 11)]
+    b = bias if with_bias else None
+    s = torch.tensor([0.0625]).bfloat16().cuda()
+    d = hip._desc(T, in_f, out_f, coef, in_f, 1, 4, torch.bfloat16, 0)
+    ref = ctypes.byref(d)
+    stream = torch.cuda.current_stream().cuda_stream
+    old = lib.rdb_set_big_tiles(2)
+    try:
+        y2, state = hip.linear_project_fwd(x, coef, 4, bias=b)
+        assert lib.rdb_linear_rbias_fwd(y2.data_ptr(), out_f, x.data_ptr(), in_f, s.data_ptr(), ref, stream) == 0
+        need = lib.rdb_linear_workspace_bytes(9, ref)
+        assert need >= in_f * out_f * 2
+        ws, y, state1 = torch.empty(need, dtype=torch.uint8, device="cuda"), torch.empty_like(y2), torch.zeros_like(state)
+
+        def call(size):
+            return lib.rdb_linear_project_fwd_rbias(y.data_ptr(), out_f, state1.data_ptr(), x.data_ptr(), in_f, coef.data_ptr(), s.data_ptr(),
+                                                    b.data_ptr() if with_bias else None, ref, ws.data_ptr(), size, stream)
+
+        assert call(need - 1) != 0 and call(need) == 0
+        again = hip.linear_fwd_projected(state1, coef, in_f, 4, bias=b)
+        first = hip.linear_fwd_projected(state, coef, in_f, 4, bias=b)
+    finally:
+        lib.rdb_set_big_tiles(old)
+    assert torch.equal(again, first)
+    N = ops.sq5_gen_2d(in_f, k, 4).double().cpu()
+    R = ops.sq5_gen_1d(in_f * out_f, 4).double().cpu().view(out_f, in_f)
+    W = coef.double().cpu() @ N.t() + 0.0625 * R
+    want = x.double().cpu() @ W.t() + (bias.double().cpu() if with_bias else 0.0)
+    err, err2 = [float((t.double().cpu() - want).norm() / want.norm()) for t in (y, y2)]
+    assert err < 8e-3 and err <= 1.02 * err2

@@ -758,15 +758,16 @@ template <typename T, int V> __global__ __launch_bounds__(NT) void column_sums_k
     }
 }
 
-// block b: coefficients b * BIAS_M .. + 3; the block behind the last coefficient: the scale
-__global__ __launch_bounds__(NT) void bias_grad_kernel(float *__restrict__ dcoef, float *__restrict__ ds, const float *__restrict__ part, int chunks, int64_t n, int64_t k,
+// block b: coefficients b * BIAS_M .. + 3; the block behind the last coefficient: the scale.  THREADS: a thread's outputs are a chain of
+// memory latencies, so long biases take blocks of 1024 (3072 outputs, k = 256: 15.7 us with 256 threads, 12 turns of the loop; vector-coef layer step 561 -> 540).
+template <int THREADS> __global__ __launch_bounds__(THREADS) void bias_grad_kernel(float *__restrict__ dcoef, float *__restrict__ ds, const float *__restrict__ part, int chunks, int64_t n, int64_t k,
                                                        uint32_t seed)
 {
-    __shared__ float sh[BIAS_M][4];
+    __shared__ float sh[BIAS_M][THREADS / 64];
     const int64_t m0 = (int64_t)blockIdx.x * BIAS_M;
     const bool scale = !dcoef || m0 >= k;
     float acc[BIAS_M] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int64_t o = threadIdx.x; o < n; o += NT) {
+    for (int64_t o = threadIdx.x; o < n; o += THREADS) {
         float g = 0.0f;
         for (int c0 = 0; c0 < chunks; c0 += 8) {   // eight loads in flight
             float v[8];
@@ -792,7 +793,9 @@ __global__ __launch_bounds__(NT) void bias_grad_kernel(float *__restrict__ dcoef
     __syncthreads();
     const int j = threadIdx.x;
     if (j >= BIAS_M) return;
-    const float v = (sh[j][0] + sh[j][1]) + (sh[j][2] + sh[j][3]);
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < THREADS / 64; w += 4) v += (sh[j][w] + sh[j][w + 1]) + (sh[j][w + 2] + sh[j][w + 3]);
     if (scale) {
         if (j == 0) ds[0] = v;
     } else if (m0 + j < k) {
@@ -834,6 +837,7 @@ extern "C" int rdb_bias_bwd(float *dcoef, float *ds, const void *dy, int dtype, 
         if (int rc = check_launch("column_sums_kernel")) return rc;
     }
     const int64_t blocks = (dcoef ? cdiv(k, BIAS_M) : 0) + (ds ? 1 : 0);
-    bias_grad_kernel<<<(unsigned)blocks, NT, 0, s>>>(dcoef, ds, part, chunks, n, k, seed);
+    if (n > 512) bias_grad_kernel<1024><<<(unsigned)blocks, 1024, 0, s>>>(dcoef, ds, part, chunks, n, k, seed);
+    else bias_grad_kernel<NT><<<(unsigned)blocks, NT, 0, s>>>(dcoef, ds, part, chunks, n, k, seed);
     return check_launch("bias_grad_kernel");
 }

@@ -558,7 +558,8 @@ template <bool DOT> __global__ __launch_bounds__(256, 1) void big_rbias_kernel(B
 // ----------------------------------------------------------------------------------------------- y = z . C^T + s * x . R^T (+ bias)
 // A forward pass with the fused random bias in one product: the tile's accumulators contract in_f (x with R), are scaled, and go on with
 // k (z with C), so that y is written once, rounded once, and never read back (8192 tokens x 768 -> 3072, k = 256: y = z . C^T beside the
-// projection and y += s x . R^T: 98 us; z, R and this: 84).  Tiles of 256 output features x 128 tokens, one persistent block a compute unit.
+// projection and y += s x . R^T: 98 us; z, R and this: 84).  Tiles of 256 output features x 128 tokens, one persistent block a compute
+// unit (256 x 256: 75 us instead of 66, the second pair of operands does not fit in registers beside 256 accumulators).
 struct BigYRParams {
     const bf16_t *noise;   // R [out_f x in_f] in fragment order
     const bf16_t *x;

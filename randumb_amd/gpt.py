@@ -137,6 +137,17 @@ class RT_Block(nn.Module):
         x, h = _add_norm(x, self.attn(RT_norm(x)))
         return x + self.mlp(h)
 
+    def _with_norm(self, x: torch.Tensor, normed: torch.Tensor):
+        """``forward`` between blocks that hand each other their output's normalisation: it and the addition are one pass over memory,
+        forwards and backwards (24 additions of 7.5 us a step of GPT-2 small otherwise)."""
+        x, h = _add_norm(x, self.attn(normed))
+        return _add_norm(x, self.mlp(h))
+
+    def _plain(self) -> bool:
+        """Nothing that has to see ``forward`` run: no subclass, no replaced method, no hooks."""
+        return (type(self) is RT_Block and "forward" not in self.__dict__ and not torch.nn.modules.module._has_any_global_hook()
+                and not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks or self._backward_pre_hooks))
+
 
 class RT_GPT(nn.Module):
     """Seeds are drawn qkv, proj, fc, mlp-proj per block, block after block."""
@@ -156,9 +167,13 @@ class RT_GPT(nn.Module):
     def forward(self, idx: torch.Tensor, target: torch.Tensor) -> torch.Tensor:
         x = self.wte(idx)
         x = RT_norm(x.to(self.h[0].mlp.c_fc.weight_coef.dtype))
+        normed = None   # RT_norm(x) where it is at hand
         for block in self.h:
-            x = block(x)
-        logits = self.lm_head(RT_norm(x))
+            if isinstance(block, RT_Block) and block._plain():
+                x, normed = block._with_norm(x, RT_norm(x) if normed is None else normed)
+            else:
+                x, normed = block(x), None
+        logits = self.lm_head(RT_norm(x) if normed is None else normed)
         ext = _fused(logits)
         if ext is not None and logits.size(-1) % 8 == 0 and logits.numel() and target.dtype is torch.int64:
             return ext.cross_entropy(logits.view(-1, logits.size(-1)), target.view(-1), -100)

@@ -125,8 +125,10 @@ class SyncWatch:
 
     def check(self, stream) -> None:
         """Waits for the work on ``stream`` and raises if any block gave up since the last look."""
-        if self.pending is None:
-            self._enqueue(stream)
+        if self.pending is not None:   # a look that tick asked for: it knows nothing of the work enqueued since
+            self.pending.synchronize()
+            self._judge()
+        self._enqueue(stream)
         self.pending.synchronize()
         self._judge()
 

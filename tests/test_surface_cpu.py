@@ -118,6 +118,43 @@ def test_sync_watch_host_logic():
         w.check(None)
 
 
+def test_explicit_look_sees_what_came_after_a_pending_one():
+    """A copy of the counter that tick has asked for says nothing of the work enqueued after it: check takes one of its own."""
+    from randumb_amd import _lib, hip
+
+    host = torch.zeros(1, dtype=torch.int32)
+
+    class Lib:
+        counter, copied, copies = 0, 0, 0
+
+        def rdb_sync_giveups_async(self, ptr, stream):
+            self.copied, self.copies = self.counter, self.copies + 1   # the value at this point of the stream
+            return 0
+
+        def rdb_set_one_launch(self, mode):
+            return 1
+
+    lib = Lib()
+
+    class Event:
+        def record(self):
+            self.value = lib.copied
+
+        def query(self):
+            return False
+
+        def synchronize(self):
+            host[0] = self.value
+
+    w = hip.SyncWatch(lib=lib, host_word=host, event_factory=Event, every=1)
+    w.tick(None)
+    assert w.pending is not None
+    lib.counter = 2   # two blocks give up behind the pending copy
+    with pytest.raises(_lib.RandumbHipError, match="2 block"):
+        w.check(None)
+    assert lib.copies == 2
+
+
 def test_big_tiles_switch_without_a_gpu():
     """rdb_set_big_tiles returns the previous mode, clamps to 0..2 and starts at 1 (the 256-wide kernels by the tile-count rule)."""
     from randumb_amd import _lib

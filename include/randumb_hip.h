@@ -174,7 +174,7 @@ enum {
 enum { RDB_OP_LINEAR_FWD = 0, RDB_OP_LINEAR_BWD_DX = 1, RDB_OP_LINEAR_BWD_DCOEF = 2, RDB_OP_LINEAR_BWD_PROJECTED = 3,
        RDB_OP_LINEAR_BWD_PROJECTED_TO = 4, RDB_OP_LINEAR_BWD_DX_DSCALE = 5, RDB_OP_LINEAR_RBIAS_BWD = 6,
        RDB_OP_LINEAR_BWD_KEPT = 7, RDB_OP_LINEAR_RBIAS_FWD = 8,
-       RDB_OP_LINEAR_PROJECT_FWD_RBIAS = 9 };
+       RDB_OP_LINEAR_PROJECT_FWD_RBIAS = 9, RDB_OP_LINEAR_RBIAS_BWD_FULL = 10 };
 
 /* Device scratch (bytes) that entry point `op` can use for `desc`; 0 when it has no use for any.  A NULL or too small
  * workspace is never an error with RDB_ALGO_AUTO: the library then runs a kernel that needs none. */
@@ -229,7 +229,8 @@ int rdb_linear_bwd_dx_dscale(void *dx, int64_t lddx, float *d_scale_bias, const 
 int rdb_linear_rbias_fwd(void *y, int64_t ldy, const void *x, int64_t ldx, const void *scale_bias,
                          const rdb_linear_desc *desc, void *stream);
 /* The same with scratch for R (rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_FWD) bytes, 16-byte aligned; less, or NULL: R is hashed
- * as the product needs it).  rdb_linear_rbias_bwd finds that scratch behind its sums. */
+ * as the product needs it).  rdb_linear_rbias_bwd takes that scratch behind its sums, in a workspace of
+ * rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_BWD_FULL) bytes, also where no d_scale_bias is wanted. */
 int rdb_linear_rbias_fwd_ws(void *y, int64_t ldy, const void *x, int64_t ldx, const void *scale_bias, const rdb_linear_desc *desc,
                             void *workspace, int64_t workspace_bytes, void *stream);
 /* rdb_linear_project_fwd and the random bias's share in one product, y = z . C^T + s * x . R^T (+ bias), rounded once.  For layers of which

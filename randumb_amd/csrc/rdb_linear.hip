@@ -477,10 +477,10 @@ static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d)
         const int64_t t = linear_dx_factored_workspace(d);
         return t > 0 ? (t + 255) / 256 * 256 + linear_dx_rbias_dot_floats(d) * 4 : 0;
     }
-    if (op == RDB_OP_LINEAR_RBIAS_BWD) {   // one float per tile of the random-bias product (the gradient of the scale); behind them R, never required
+    if (op == RDB_OP_LINEAR_RBIAS_BWD || op == RDB_OP_LINEAR_RBIAS_BWD_FULL) {   // one float per tile of the random-bias product (the gradient of the scale)
         if (d->act_dtype != RDB_BF16 || d->coef_dtype != RDB_BF16 || d->in_f % 8 || d->out_f % 8) return 0;
-        const int64_t table = rbias_big_table_bytes(d, d->in_f, num_compute_units());
-        return table > 0 ? rbias_dot_room(d) + table : linear_dx_rbias_dot_floats(d) * 4;
+        const int64_t table = op == RDB_OP_LINEAR_RBIAS_BWD_FULL ? rbias_big_table_bytes(d, d->in_f, num_compute_units()) : 0;
+        return table > 0 ? rbias_dot_room(d) + table : linear_dx_rbias_dot_floats(d) * 4;   // ... and R behind them
     }
     if (op == RDB_OP_LINEAR_PROJECT_FWD_RBIAS) return project_fwd_rbias_table(d);
     if (op == RDB_OP_LINEAR_RBIAS_FWD)

@@ -409,7 +409,7 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         if (has_sb && dx.defined()) {
             const Tensor x = act(saved[3]), sb = native(scale_bias).to(at::kBFloat16);
             const rdb_linear_desc r = rbias_desc(dy, l);
-            const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_BWD, &r);
+            const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_BWD_FULL, &r);
             const Tensor ws = bytes(need, dy);
             if (want_sb) {
                 dsb = at::empty({1}, dy.options().dtype(at::kFloat));

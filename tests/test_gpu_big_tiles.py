@@ -309,7 +309,7 @@ def test_random_bias_from_memory(T, in_f, out_f):
         dots = -(-in_f // 64) * -(-T // 256) * 4
         out = []
         for table in (True, False):
-            fwd, bwd = [lib.rdb_linear_workspace_bytes(op, ref) if table else n for op, n in ((8, 0), (6, dots))]
+            fwd, bwd = [lib.rdb_linear_workspace_bytes(op, ref) if table else n for op, n in ((8, 0), (10, dots))]
             if table:
                 assert fwd >= in_f * out_f * 2 and bwd >= dots + in_f * out_f * 2
             y, dx, dx_only, ds = y0.clone(), dx0.clone(), dx0.clone(), torch.empty(1, device="cuda")

@@ -39,6 +39,22 @@ __global__ __launch_bounds__(256) void f32_sum_scalars_kernel(float *__restrict_
     if (threadIdx.x == 0) out[0] = sh[0];
 }
 
+// part[0] + part[stride] + ... in split order, eight loads in flight: one at a time the sum is a chain of `splits` memory latencies
+// (4097 tokens x 1001 -> 999 in bf16, k = 100: step 97 -> 91 us, three of these launches)
+template <typename V> __device__ __forceinline__ V sum_in_order(const float *__restrict__ part, int64_t stride, int splits)
+{
+    V v = *reinterpret_cast<const V *>(part);
+    for (int s0 = 1; s0 < splits; s0 += 8) {
+        V u[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) u[j] = *reinterpret_cast<const V *>(part + (int64_t)min(s0 + j, splits - 1) * stride);   // clamped: loaded, not added
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (s0 + j < splits) v += u[j];
+    }
+    return v;
+}
+
 // out[i] = part[0][i] + part[1][i] + ... in split order, four values per thread (n4 groups of four, then the n % 4 last values
 // one thread each); out fp32, or bf16 (rounded once)
 __global__ __launch_bounds__(256) void f32_sum_splits_kernel(void *__restrict__ out, int out_bf16, const float *__restrict__ part, int64_t n, int64_t stride,
@@ -46,14 +62,12 @@ __global__ __launch_bounds__(256) void f32_sum_splits_kernel(void *__restrict__ 
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, n4 = vec ? n / 4 : 0;
     if (i < n4) {
-        f32x4 v = *reinterpret_cast<const f32x4 *>(part + i * 4);
-        for (int s = 1; s < splits; ++s) v += *reinterpret_cast<const f32x4 *>(part + s * stride + i * 4);
+        const f32x4 v = sum_in_order<f32x4>(part + i * 4, stride, splits);
         if (out_bf16) store4<bf16_t>(static_cast<bf16_t *>(out) + i * 4, v[0], v[1], v[2], v[3]);
         else *reinterpret_cast<f32x4 *>(static_cast<float *>(out) + i * 4) = v;
     } else if (n4 * 4 + (i - n4) < n) {
         const int64_t e = n4 * 4 + (i - n4);
-        float v = part[e];
-        for (int s = 1; s < splits; ++s) v += part[s * stride + e];
+        const float v = sum_in_order<float>(part + e, stride, splits);
         if (out_bf16) static_cast<bf16_t *>(out)[e] = f32_to_bf16(v);
         else static_cast<float *>(out)[e] = v;
     }
@@ -234,8 +248,9 @@ int linear_dcoef_f32(float *dcoef, float *d_scale_bias, const void *dy, int64_t 
 // fp32 with k <= 64: where the kernels above are ahead of the vector-ALU kernels of rdb_smallk.hip.  Microseconds of one direction
 // (contraction over J, expansion to E columns), fitted to 252 measured calls (k 16, 32, 64; 32 to 1024 tokens; 128 -> 256 to
 // 4096 -> 11008): what it picks is 0.2 us behind the faster of the two on average.  The vector-ALU kernels' hash costs a wave 0.2 us a
-// coefficient whatever the tokens, and their time grows with the products; the matrix cores' grows with the contraction a
-// block walks through alone.  1024 tokens x 4096 -> 11008, k = 64: forward 134 -> 41 us, dx 93 -> 45; 128 tokens x 784 -> 256,
+// coefficient whatever the tokens (0.16 since they fetch all their coefficients at once: up to 3 us less at k = 64 than the model
+// says, so a call near the line may now be 2 us behind), and their time grows with the products; the matrix cores' grows with
+// the contraction a block walks through alone.  1024 tokens x 4096 -> 11008, k = 64: forward 134 -> 41 us, dx 93 -> 45; 128 tokens x 784 -> 256,
 // k = 64: 20.4 -> 18.8, 20.8 -> 15.8; k = 16 stays (10.5 against 16.2).
 static double few_token_us(const rdb_linear_desc *d)
 {

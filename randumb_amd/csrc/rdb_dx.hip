@@ -11,8 +11,11 @@
 // src/rten_cpp/RandumbTensor.py:942-946).
 #include "rdb_blocks.hpp"
 #include "rdb_stationary.hpp"
+#include <algorithm>
 
 namespace rdb {
+
+int num_compute_units();   // rdb_error.hip
 
 constexpr int X_BK = 64;
 
@@ -50,28 +53,70 @@ struct DyCParams {
     int64_t lddy;
     int tokens, out_f, k;
     int tiles_c, tiles_t;
+    // the contraction is added up in `ranges` ranges of range_len output features, range by range, whoever computes them.  part == NULL:
+    // every block runs its tile's ranges one after the other; else a block per tile and range, whose sums go to
+    // part[range][token][coefficient] for dyc_sum_kernel
+    float *part;
+    int ranges, range_len;
     int frag_ksteps;  // 0: t row-major [tokens x k]; else t in fragment order with this many k-steps per 32 tokens and scaled
                       // by 2^-31, for the kernel that keeps it in registers (rdb_stationary.hpp)
 };
 
+// A range's sums, waves as WM x (4 / WM): four consecutive coefficients of a token a lane and store
+template <int MI, int NI, int WM>
+__device__ __forceinline__ void dyc_store_part(const DyCParams &p, const f32x16 (&acc)[MI][NI], int range, int m0, int tok0)
+{
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5, wm = wave / (4 / WM), wn = wave % (4 / WM);
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) {
+        const int tok = tok0 + wn * NI * 32 + ni * 32 + r;
+        if (tok >= p.tokens) continue;
+        float *row = p.part + ((int64_t)range * p.tokens + tok) * p.k;
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int jq = 0; jq < 4; ++jq) {
+                const int m = m0 + wm * MI * 32 + mi * 32 + 8 * jq + 4 * g;
+                if (m < p.k)   // k is a multiple of 8
+                    *reinterpret_cast<f32x4 *>(row + m) = f32x4{acc[mi][ni][jq * 4], acc[mi][ni][jq * 4 + 1], acc[mi][ni][jq * 4 + 2], acc[mi][ni][jq * 4 + 3]};
+            }
+    }
+}
+
 // `block`: index of this block among the blocks that run this body.
 __device__ __forceinline__ void dyc_block(const DyCParams &p, bf16_t *lds, int block)
 {
-    // work item = (token tile, coefficient tile), coefficient tile fastest: neighbours share the dy tile
-    const int w = xcd_work_item(block, p.tiles_c * p.tiles_t);
-    if (w >= p.tiles_c * p.tiles_t) return;
+    // work item = (range, token tile, coefficient tile), coefficient tile fastest: neighbours share the dy tile
+    const int tiles = p.tiles_c * p.tiles_t, items = p.part ? tiles * p.ranges : tiles, wr = xcd_work_item(block, items);
+    if (wr >= items) return;
+    const int range = wr / tiles, w = wr - range * tiles, last = p.part ? range : p.ranges - 1;
     const int m0 = (w % p.tiles_c) * K1_BC, tok0 = (w / p.tiles_c) * K1_BT;
-    f32x16 acc[K1_BC / 64][K1_BT / 64];
+    f32x16 acc[K1_BC / 64][K1_BT / 64], sum[K1_BC / 64][K1_BT / 64];
+    for (int rg = range; rg <= last; ++rg) {
+        const int o_begin = rg * p.range_len, o_end = min(p.out_f, o_begin + p.range_len);
 #pragma unroll
-    for (int mi = 0; mi < K1_BC / 64; ++mi)
+        for (int mi = 0; mi < K1_BC / 64; ++mi)
 #pragma unroll
-        for (int ni = 0; ni < K1_BT / 64; ++ni) acc[mi][ni] = zero16();
-    // "A": C[o][m], tile rows = m (contiguous in memory), contraction index = o
-    GlobalOperand<K1_BC, X_BK, M_CONT> opc = {p.coef, (int64_t)p.k, m0, p.k, p.out_f, (int64_t)p.out_f * p.k};
-    // "B": dy[tok][o], contraction index contiguous
-    GlobalOperand<K1_BT, X_BK, K_CONT> opdy = {p.dy, p.lddy, tok0, p.tokens, p.out_f, (int64_t)(p.tokens - 1) * p.lddy + p.out_f};
-    gemm_mainloop<K1_BC, K1_BT, X_BK, 2, 2>(acc, lds, opc, opdy, 0, (p.out_f + X_BK - 1) / X_BK);
-    if (p.frag_ksteps)
+            for (int ni = 0; ni < K1_BT / 64; ++ni) acc[mi][ni] = zero16();
+        // "A": C[o][m], tile rows = m (contiguous in memory), contraction index = o
+        GlobalOperand<K1_BC, X_BK, M_CONT> opc = {p.coef, (int64_t)p.k, m0, p.k, o_end, (int64_t)p.out_f * p.k};
+        // "B": dy[tok][o], contraction index contiguous
+        GlobalOperand<K1_BT, X_BK, K_CONT> opdy = {p.dy, p.lddy, tok0, p.tokens, o_end, (int64_t)(p.tokens - 1) * p.lddy + p.out_f};
+        gemm_mainloop<K1_BC, K1_BT, X_BK, 2, 2>(acc, lds, opc, opdy, o_begin, (o_end - o_begin + X_BK - 1) / X_BK);
+        if (last == range) break;
+        __syncthreads();   // the next range begins by writing the stage buffers
+#pragma unroll
+        for (int mi = 0; mi < K1_BC / 64; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < K1_BT / 64; ++ni) {
+                if (rg > range) sum[mi][ni] += acc[mi][ni];
+                else sum[mi][ni] = acc[mi][ni];
+                acc[mi][ni] = sum[mi][ni];
+            }
+    }
+    if (p.part)
+        dyc_store_part<K1_BC / 64, K1_BT / 64, 2>(p, acc, range, m0, tok0);
+    else if (p.frag_ksteps)
         store_tile_bf16_frag<K1_BC, K1_BT>(acc, lds, p.t, p.frag_ksteps, m0, p.frag_ksteps * 16, tok0, (p.tokens + 31) / 32 * 32,
                                            4.656612873077392578125e-10f);
     else
@@ -83,27 +128,77 @@ __device__ __forceinline__ void dyc_block(const DyCParams &p, bf16_t *lds, int b
 // the coefficient rows (one 32-row block each, no fragment loaded twice) and share the 64 tokens.
 __device__ __forceinline__ void dyc_block_direct(const DyCParams &p, bf16_t *lds, int block)
 {
-    const int w = xcd_work_item(block, p.tiles_c * p.tiles_t);
-    if (w >= p.tiles_c * p.tiles_t) return;
+    const int tiles = p.tiles_c * p.tiles_t, items = p.part ? tiles * p.ranges : tiles, wr = xcd_work_item(block, items);
+    if (wr >= items) return;
+    const int range = wr / tiles, w = wr - range * tiles, last = p.part ? range : p.ranges - 1;
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int m0 = (w % p.tiles_c) * K1_BC, tok0 = (w / p.tiles_c) * K1_BT;
-    f32x16 acc[1][K1_BT / 32];
-#pragma unroll
-    for (int ni = 0; ni < K1_BT / 32; ++ni) acc[0][ni] = zero16();
+    f32x16 acc[1][K1_BT / 32], sum[K1_BT / 32];
     // stages of 128: half as many barriers (and waits for the first fragments after them) as with 64, for the same LDS
     constexpr int BKD = RDB_DYC_BKD;
-    GlobalOperand<K1_BT, BKD, K_CONT> opdy = {p.dy, p.lddy, tok0, p.tokens, p.out_f, (int64_t)(p.tokens - 1) * p.lddy + p.out_f};
     FragSource fc;
     fc.init(p.ctf, (int64_t)p.kpad * p.osteps * 16, p.osteps, (m0 >> 5) + wave, lane);
     // these blocks are the longer ones of the launch they share with the coefficient-gradient blocks: their waves issue first
     __builtin_amdgcn_s_setprio(RDB_DYC_PRIO);
-    direct_mainloop<K1_BT / 32, 1, BKD / 16, false, RDB_DYC_TRIP, RDB_DYC_DSTG, RDB_DYC_RD>(acc, lds, opdy, fc, 0, (p.out_f + BKD - 1) / BKD, 0, lane);
-    if (p.frag_ksteps)
+    for (int rg = range; rg <= last; ++rg) {
+        const int o_begin = rg * p.range_len, o_end = min(p.out_f, o_begin + p.range_len);
+#pragma unroll
+        for (int ni = 0; ni < K1_BT / 32; ++ni) acc[0][ni] = zero16();
+        GlobalOperand<K1_BT, BKD, K_CONT> opdy = {p.dy, p.lddy, tok0, p.tokens, o_end, (int64_t)(p.tokens - 1) * p.lddy + p.out_f};
+        direct_mainloop<K1_BT / 32, 1, BKD / 16, false, RDB_DYC_TRIP, RDB_DYC_DSTG, RDB_DYC_RD>(acc, lds, opdy, fc, o_begin, (o_end - o_begin + BKD - 1) / BKD, 0,
+                                                                                               lane);
+        if (last == range) break;
+        __syncthreads();   // the next range begins by writing the stage buffers
+#pragma unroll
+        for (int ni = 0; ni < K1_BT / 32; ++ni) {
+            if (rg > range) sum[ni] += acc[0][ni];
+            else sum[ni] = acc[0][ni];
+            acc[0][ni] = sum[ni];
+        }
+    }
+    if (p.part)
+        dyc_store_part<1, K1_BT / 32, 4>(p, acc, range, m0, tok0);
+    else if (p.frag_ksteps)
         store_tile_bf16_frag<K1_BC, K1_BT, 4>(acc, lds, p.t, p.frag_ksteps, m0, p.frag_ksteps * 16, tok0, (p.tokens + 31) / 32 * 32,
                                               4.656612873077392578125e-10f);
     else
         store_tile_bf16<K1_BC, K1_BT, 4>(acc, lds, p.t, p.k, m0, p.k, tok0, p.tokens, 1.0f, nullptr);
     RDB_STAMP(3);
+}
+
+// t from the ranges' sums, added in range order: eight coefficients of a token a thread, in fragment order (as store_tile_bf16_frag
+// writes it: tokens padded to 32 and coefficients to a multiple of 64 with zeros, times 2^-31)
+__global__ __launch_bounds__(256) void dyc_sum_kernel(DyCParams p, int pieces, int k8)
+{
+    const int e = (int)blockIdx.x * 256 + threadIdx.x;
+    if (e >= pieces) return;
+    const int tok = e / k8, m = (e - tok * k8) * 8;
+    f32x4 lo = {0.0f, 0.0f, 0.0f, 0.0f}, hi = lo;
+    if (tok < p.tokens && m < p.k) {
+        const float *src = p.part + (int64_t)tok * p.k + m;
+        const int64_t stride = (int64_t)p.tokens * p.k;
+        f32x4 a[8], b[8];   // at most eight ranges, all in flight
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float *q = src + (int64_t)min(i, p.ranges - 1) * stride;
+            a[i] = *reinterpret_cast<const f32x4 *>(q);
+            b[i] = *reinterpret_cast<const f32x4 *>(q + 4);
+        }
+        lo = a[0];
+        hi = b[0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i)
+            if (i < p.ranges) {
+                lo += a[i];
+                hi += b[i];
+            }
+    }
+    lo *= 4.656612873077392578125e-10f;
+    hi *= 4.656612873077392578125e-10f;
+    bf16_t *dst = p.t + ((int64_t)(tok >> 5) * p.frag_ksteps + (m >> 4)) * 512 + (((m >> 3) & 1) * 32 + (tok & 31)) * 8;
+    const i32x4 h = {(int)f32x2_to_bf16x2(lo[0], lo[1]), (int)f32x2_to_bf16x2(lo[2], lo[3]), (int)f32x2_to_bf16x2(hi[0], hi[1]),
+                     (int)f32x2_to_bf16x2(hi[2], hi[3])};
+    *reinterpret_cast<i32x4 *>(dst) = h;
 }
 
 __global__ __launch_bounds__(256, 2) void dx_dyc_kernel(DyCParams p)
@@ -239,6 +334,19 @@ int64_t linear_bwd_projected_workspace(const rdb_linear_desc *d, int num_cus, bo
     return align256(linear_dx_factored_workspace(d)) + (int64_t)dc.splits * d->out_f * d->k * (int64_t)sizeof(float);
 }
 
+// Ranges of t = dy . C where its tiles are half the compute units or fewer and each contracts 2048 output features or more: a block walks
+// through them at 1 us a stage of 128 while the launch's other blocks are long done (1178 tokens x 640 -> 6520, k = 160: 38 blocks of 51
+// stages; the whole backward pass 57 -> 30 us with the launch that adds the ranges up; 2048 x 4096 -> 11008, k = 256: 91 -> 61).  At least 1024 output features a range, at most eight.  k <= 256 only: the
+// 256-wide tiles, which take longer ones where there are enough of them, contract in one range, and both give the same bits.  The rule
+// knows nothing of workspaces: without room for the ranges' sums a block adds its tile's ranges up itself, to the same bits.
+static int dyc_ranges(const rdb_linear_desc *d, int num_cus, int *range_len)
+{
+    const int64_t tiles = cdiv(d->k, K1_BC) * cdiv(d->tokens, K1_BT);
+    int64_t r = std::min<int64_t>(std::min<int64_t>(num_cus / tiles, d->out_f / 1024), 8);
+    if (r < 2 || d->k > ST_KMAX) r = 1;
+    *range_len = (int)(cdiv(cdiv(d->out_f, r), 128) * 128);
+    return (int)cdiv(d->out_f, *range_len);
+}
 static void make_dyc_params(DyCParams &p1, const void *dy, int64_t lddy, const void *coef, void *t, const rdb_linear_desc *d)
 {
     p1.dy = (const bf16_t *)dy;
@@ -256,7 +364,18 @@ static void make_dyc_params(DyCParams &p1, const void *dy, int64_t lddy, const v
     p1.k = (int)d->k;
     p1.tiles_c = (int)cdiv(d->k, K1_BC);
     p1.tiles_t = (int)cdiv(d->tokens, K1_BT);
+    p1.part = nullptr;
+    p1.ranges = dyc_ranges(d, num_compute_units(), &p1.range_len);
     p1.frag_ksteps = 0;
+}
+
+// Scratch of the regrouped backward pass that it can do without: the ranges' sums, and later, in their place, N^T for dx = t . N
+int64_t linear_bwd_projected_extra(const rdb_linear_desc *d, int num_cus)
+{
+    if (!dx_factored_ok(d)) return 0;
+    int len;
+    const int ranges = dyc_ranges(d, num_cus, &len);
+    return std::max<int64_t>(ranges > 1 ? align256(ranges * d->tokens * d->k * (int64_t)sizeof(float)) : 0, dx_big_table_bytes(d, num_cus));
 }
 
 // t . N with t in registers applies when k is short enough and dx fits a buffer descriptor.
@@ -353,6 +472,11 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             a.dyc.kpad = L.kpad;
         }
         if (tn_stationary_ok(d, lddx)) a.dyc.frag_ksteps = (int)cdiv(d->k, 64) * 4;   // the t.N kernel below keeps t in registers
+        const int64_t base = align256(linear_bwd_projected_workspace(d, num_cus, accumulate || dc_bf16));
+        if (a.dyc.frag_ksteps) {
+            if (a.dyc.ranges > 1 && workspace_bytes >= base + align256(a.dyc.ranges * d->tokens * d->k * (int64_t)sizeof(float)))
+                a.dyc.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + base);
+        }
         a.dc_blocks = xcd_grid_size(dc_items);
         int rc = RDB_OK;
         const int red_splits = big ? 1 : a.dc.splits;
@@ -364,8 +488,13 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
         } else {
             size_t smem = smem_dc > smem_dyc ? smem_dc : smem_dyc;
             if (int rl = reserve_lds(reinterpret_cast<const void *>(bwd_dc_dyc_kernel), smem, "bwd_dc_dyc_kernel")) return rl;
-            bwd_dc_dyc_kernel<<<a.dc_blocks + xcd_grid_size(p1.tiles_c * p1.tiles_t), 256, smem, s>>>(a);
+            bwd_dc_dyc_kernel<<<a.dc_blocks + xcd_grid_size(p1.tiles_c * p1.tiles_t * (a.dyc.part ? a.dyc.ranges : 1)), 256, smem, s>>>(a);
             rc = check_launch("bwd_dc_dyc_kernel");
+            if (!rc && a.dyc.part) {
+                const int k8 = a.dyc.frag_ksteps * 2, pieces = (int)(cdiv(d->tokens, 32) * 32) * k8;
+                dyc_sum_kernel<<<(unsigned)cdiv(pieces, 256), 256, 0, s>>>(a.dyc, pieces, k8);
+                rc = check_launch("dyc_sum_kernel");
+            }
         }
         if (rc) return rc;
         if (!(g_bwd_parts & 2)) return RDB_OK;
@@ -402,7 +531,7 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             }
             return check_launch("bwd_tns_red_kernel");
         }
-        const int64_t table = dx_big_table_bytes(d, num_cus), base = align256(linear_bwd_projected_workspace(d, num_cus, accumulate || dc_bf16));
+        const int64_t table = dx_big_table_bytes(d, num_cus);
         if (direct && table && workspace_bytes >= base + table) {   // nothing to add up, and room for N^T
             rc = linear_tn_big(dx, lddx, workspace, static_cast<char *>(workspace) + base, d, num_cus, s);
             if (rc != RDB_E_UNSUPPORTED) return rc;

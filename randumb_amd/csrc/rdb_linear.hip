@@ -346,7 +346,7 @@ int big_tiles_mode();
 bool big_bwd_applies(const rdb_linear_desc *d, int num_cus);
 int linear_bwd_big(void *t, void *dc, bool dc_bf16, const void *dy, int64_t lddy, const void *state, const void *coef, const rdb_linear_desc *d,
                    int num_cus, bool want_t, bool want_dc, hipStream_t s);
-int64_t dx_big_table_bytes(const rdb_linear_desc *d, int num_cus);
+int64_t linear_bwd_projected_extra(const rdb_linear_desc *d, int num_cus);
 
 // rdb_rbias.hip
 int linear_dx_rbias_add(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table = nullptr, int64_t table_bytes = 0);
@@ -405,7 +405,7 @@ template <typename K> static int launch(K kernel, dim3 grid, size_t smem, hipStr
 using namespace rdb;
 
 static int64_t bwd_projected_workspace(const rdb_linear_desc *d, bool force_partial);
-static int64_t bwd_projected_table(const rdb_linear_desc *d);
+static int64_t bwd_projected_extra(const rdb_linear_desc *d);
 static int64_t project_fwd_rbias_table(const rdb_linear_desc *d);
 
 // vector-coef coefficient gradient in two passes: dW = dy^T . x into the workspace (and the partial matrices of its token
@@ -486,8 +486,8 @@ static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d)
     if (op == RDB_OP_LINEAR_RBIAS_FWD)
         return d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16 ? rbias_big_table_bytes(d, d->out_f, num_compute_units()) : 0;
     if (op == RDB_OP_LINEAR_BWD_PROJECTED || op == RDB_OP_LINEAR_BWD_PROJECTED_TO) {
-        const int64_t base = bwd_projected_workspace(d, op == RDB_OP_LINEAR_BWD_PROJECTED_TO), table = base > 0 ? bwd_projected_table(d) : 0;
-        return table > 0 ? (base + 255) / 256 * 256 + table : base;   // what lies behind `base` is never required
+        const int64_t base = bwd_projected_workspace(d, op == RDB_OP_LINEAR_BWD_PROJECTED_TO), extra = base > 0 ? bwd_projected_extra(d) : 0;
+        return extra > 0 ? (base + 255) / 256 * 256 + extra : base;   // what lies behind `base` is never required
     }
     if (op == RDB_OP_LINEAR_FWD) return d->coef_dtype == RDB_BF16 ? linear_projection_bytes(d) : 0;
     if (op == RDB_OP_LINEAR_BWD_DCOEF) return linear_projection_bytes(d);  // reads no coefficients: their dtype does not matter
@@ -1188,8 +1188,8 @@ static int64_t bwd_projected_workspace(const rdb_linear_desc *d, bool force_part
     const rdb_linear_desc first = chunk_desc(d, pl, 0);
     return linear_bwd_projected_workspace(&first, num_compute_units(), pl.nchunks > 1 || force_partial);
 }
-// N^T for dx = t . N of a layer that runs as one chunk of tokens (the chunks after the first have their sums added up beside that product)
-static int64_t bwd_projected_table(const rdb_linear_desc *d) { return chunk_plan(d).nchunks == 1 ? dx_big_table_bytes(d, num_compute_units()) : 0; }
+// Scratch that a layer that runs as one chunk of tokens can use beyond that and do without
+static int64_t bwd_projected_extra(const rdb_linear_desc *d) { return chunk_plan(d).nchunks == 1 ? linear_bwd_projected_extra(d, num_compute_units()) : 0; }
 
 static int bwd_projected_entry(const char *who, void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, const void *dy, int64_t lddy, const void *z,
                                const void *coef, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)

@@ -65,3 +65,34 @@ def test_spread_projection_replayed_from_a_graph(hip):
         assert torch.equal(y, want[i]), i
         assert torch.equal(hip.linear_project_fwd(xs[i], C, 7)[0], want[i])
     hip.sync_check()
+
+
+@pytest.mark.parametrize("T,in_f,out_f,k", [(300, 264, 2056, 72), (1178, 136, 6520, 160), (70, 64, 8200, 248), (129, 72, 3080, 256)])
+@pytest.mark.parametrize("with_ct", [True, False])
+def test_split_dy_product(T, in_f, out_f, k, with_ct):
+    """t = dy . C in ranges of the output features (few tiles, long rows of dy): against float64, and the same bits
+    twice, with a workspace that has no room for the ranges' sums, and from the input gradient's own entry point."""
+    import ctypes
+
+    from randumb_amd import _lib, hip, ops
+
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(T)
+    x, dy = torch.randn(T, in_f, generator=g).bfloat16().cuda(), torch.randn(T, out_f, generator=g).bfloat16().cuda()
+    c = (torch.randn(out_f, k, generator=g) / k ** 0.5).bfloat16().cuda()
+    ref = ctypes.byref(hip._desc(T, in_f, out_f, c, in_f, 1, 5, torch.bfloat16, 0))
+    state = hip.linear_project(x, k, out_f, 5, coef=c if with_ct else None)
+    full, part = lib.rdb_linear_workspace_bytes(4, ref), T * k * 4
+    out = []
+    for size in (full, full, full - 2 * part):
+        dx, dc, ws = torch.empty_like(x), torch.empty_like(c), torch.empty(size, dtype=torch.uint8, device="cuda")
+        assert lib.rdb_linear_bwd_projected_to(dx.data_ptr(), in_f, dc.data_ptr(), 1, dy.data_ptr(), out_f, state.data_ptr(), c.data_ptr(), ref,
+                                               ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream) == 0
+        out.append((dx, dc))
+    for dx, dc in out[1:]:
+        assert torch.equal(dx, out[0][0]) and torch.equal(dc, out[0][1])
+    assert torch.equal(hip.linear_bwd_dx(dy, c, in_f, out_f, in_f, 1, 5, algo=_lib.RDB_ALGO_FACTORED), out[0][0])
+    N = ops.sq5_gen_2d(in_f, k, 5).double().cpu()
+    want = (dy.double().cpu() @ c.double().cpu()) @ N.t()
+    assert float((out[0][0].double().cpu() - want).norm() / want.norm()) < 8e-3
+    assert float((out[0][1].double().cpu() - dy.double().cpu().t() @ (x.double().cpu() @ N)).norm() / (dy.double().cpu().t() @ (x.double().cpu() @ N)).norm()) < 8e-3

@@ -336,9 +336,11 @@ int64_t linear_bwd_projected_workspace(const rdb_linear_desc *d, int num_cus, bo
 
 // Ranges of t = dy . C where its tiles are half the compute units or fewer and each contracts 2048 output features or more: a block walks
 // through them at 1 us a stage of 128 while the launch's other blocks are long done (1178 tokens x 640 -> 6520, k = 160: 38 blocks of 51
-// stages; the whole backward pass 57 -> 30 us with the launch that adds the ranges up; 2048 x 4096 -> 11008, k = 256: 91 -> 61).  At least 1024 output features a range, at most eight.  k <= 256 only: the
-// 256-wide tiles, which take longer ones where there are enough of them, contract in one range, and both give the same bits.  The rule
-// knows nothing of workspaces: without room for the ranges' sums a block adds its tile's ranges up itself, to the same bits.
+// stages; the whole backward pass 57 -> 30 us with the launch that adds the ranges up; 2048 x 4096 -> 11008, k = 256: 91 -> 61; at the
+// line, 300 x 512 -> 2048, k = 64: 21.7 -> 20.0, 2048 x 1024 -> 2048, k = 96: 19.1 -> 18.5).  At least 1024 output features a range, at
+// most eight ranges.  k <= 256 only: the 256-wide tiles, which take longer ones where there are enough of them, contract in one range,
+// and both give the same bits.  The rule knows nothing of workspaces: without room for the ranges' sums a block adds its tile's
+// ranges up itself, to the same bits.
 static int dyc_ranges(const rdb_linear_desc *d, int num_cus, int *range_len)
 {
     const int64_t tiles = cdiv(d->k, K1_BC) * cdiv(d->tokens, K1_BT);

@@ -49,6 +49,8 @@ struct ZParams {
     int ranges, range_stages;
     char *part;
     SyncWait sync_wait;
+    // C's transposition: by the projecting blocks, after their tiles, or (c_blocks > 0) by that many blocks behind the z_grid projecting ones
+    int z_grid, c_blocks;
 };
 
 // Eight waves, two to a SIMD: the tile's noise is hashed once per stage by all 512 threads (4 values each) on the vector ALU,
@@ -56,6 +58,29 @@ struct ZParams {
 // x pieces (loaded two stages ahead) and the next stage's noise go registers -> LDS, 4 MFMAs per wave (its 32 tokens), one
 // barrier.  Written without the 256-thread tile engine; the LDS layouts and fragment reads are the engine's (OperandTile).
 constexpr int KZ_THREADS = 512;
+
+// C transposed into fragment order by blocks of their own, two 1 KB units (see z_block) a wave and turn.  For layers whose projecting blocks
+// leave compute units free: those took 1.5 us a unit, one after the other, before anybody saw their tiles (1178 tokens x 640 -> 6520,
+// k = 160: 25 blocks with 12 units a wave; forward 26 -> 20 us; 512 x 1024 -> 4096, k = 128: 24.4 -> 18.5).
+__device__ __forceinline__ void transpose_units(const ZParams &p, int first, int step)
+{
+    const int lane = threadIdx.x & 63, osteps = p.out64 >> 4, units = (p.kpad >> 5) * osteps;
+    for (int u0 = first; u0 < units; u0 += 2 * step) {
+        uint32_t w[2][8];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int u = min(u0 + i * step, units - 1), mb = u / osteps, m = mb * 32 + (lane & 31), o0 = (u - mb * osteps) * 16 + (lane >> 5) * 8;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) w[i][j] = (m < p.k && o0 + j < p.out_f) ? p.coef[(int64_t)(o0 + j) * p.k + m] : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if (u0 + i * step >= units) break;
+            const i32x4 v = {(int)(w[i][0] | (w[i][1] << 16)), (int)(w[i][2] | (w[i][3] << 16)), (int)(w[i][4] | (w[i][5] << 16)), (int)(w[i][6] | (w[i][7] << 16))};
+            store_stream(reinterpret_cast<i32x4 *>(p.ctf + (int64_t)(u0 + i * step) * 512 + lane * 8), v);
+        }
+    }
+}
 
 // `block` of `nblocks`: index of this block among the blocks that run this body; all KZ_THREADS threads must call.  RANGES: the
 // contraction may be in several ranges; a kernel of its own for the ordinary case, whose 128 registers let two blocks share a
@@ -71,7 +96,7 @@ template <bool RANGES> __device__ __forceinline__ void z_block(const ZParams &p,
     // C transposed into fragment order, a 1 KB unit (32 coefficients x 16 output features) per wave and turn: lane (r, g)
     // gathers C[o0 + 8 g + j][m0 + r], j = 0..7 (32 lanes read 64 consecutive bytes of a row) and stores its 16 bytes.
     // The first turn's loads are issued here and stored after the tile's main loop, which hides their latency.
-    const int osteps = p.out64 >> 4, units = p.coef ? (p.kpad >> 5) * osteps : 0;
+    const int osteps = p.out64 >> 4, units = p.coef && !p.c_blocks ? (p.kpad >> 5) * osteps : 0;
     auto gather_unit = [&](int u, uint32_t (&w)[8]) {   // the raw values: combining them would wait for the loads
         const int mb = u / osteps, os = u % osteps, m = mb * 32 + (lane & 31);
 #pragma unroll
@@ -294,7 +319,8 @@ template <bool RANGES> __device__ __forceinline__ void z_block(const ZParams &p,
 template <bool RANGES> __global__ __launch_bounds__(KZ_THREADS, 1) void factored_z_kernel(ZParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    z_block<RANGES>(p, smem_raw, blockIdx.x, gridDim.x);
+    if ((int)blockIdx.x < p.z_grid) z_block<RANGES>(p, smem_raw, blockIdx.x, p.z_grid);
+    else transpose_units(p, ((int)blockIdx.x - p.z_grid) * (KZ_THREADS / 64) + (int)(threadIdx.x >> 6), p.c_blocks * (KZ_THREADS / 64));
 }
 
 // ----------------------------------------------------------------------------------------------- y = z . C^T
@@ -342,23 +368,25 @@ template <int KG, bool BIAS> __global__ __launch_bounds__(ST_THREADS, 1) void fa
     stationary_block<KG, BIAS, false, true>(p, smem_raw, blockIdx.x);
 }
 
-// Projection and forward product in one launch: blocks 0 .. z_blocks - 1 project (z_block), the others multiply
-// (stationary_block) and wait, tile by tile, for the tags of the projection blocks that feed them.  A multiplying block
+// Projection and forward product in one launch: blocks 0 .. z_grid - 1 project (z_block), the next c_blocks transpose C, the others multiply
+// (stationary_block; z_grid and c_blocks are multiples of 8, so that all kinds keep their numbering over the dies) and wait, tile by tile, for the tags of the projection blocks that feed them.  A multiplying block
 // starts on a compute unit the moment a projecting block leaves it: no drain of the whole chip, no second launch in between.
 struct ZYParams {
     ZParams z;
     StParams y;
-    int z_blocks;   // a multiple of 8, so that both kinds keep their numbering over the dies
 };
 
 template <int KG, bool BIAS> __global__ __launch_bounds__(ST_THREADS, 1) void factored_zy_kernel(ZYParams p)
 {
     static_assert(KZ_THREADS == ST_THREADS && KZ_BT == ST_BT, "one block size and one token tile for both kinds of block");
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    if ((int)blockIdx.x < p.z_blocks)
-        z_block<true>(p.z, smem_raw, blockIdx.x, p.z_blocks);
+    const int block = (int)blockIdx.x - p.z.z_grid;
+    if (block < 0)
+        z_block<true>(p.z, smem_raw, blockIdx.x, p.z.z_grid);
+    else if (block < p.z.c_blocks)
+        transpose_units(p.z, block * (KZ_THREADS / 64) + (int)(threadIdx.x >> 6), p.z.c_blocks * (KZ_THREADS / 64));
     else
-        stationary_block<KG, BIAS, false, true>(p.y, smem_raw, blockIdx.x - p.z_blocks);
+        stationary_block<KG, BIAS, false, true>(p.y, smem_raw, block - p.z.c_blocks);
 }
 
 // ----------------------------------------------------------------------------------------------- dC = dy^T . z
@@ -441,6 +469,8 @@ static bool fill_z_params(ZParams &p, void *state, const void *x, int64_t ldx, c
     p.sync = nullptr;
     p.sync_tag = 0;
     p.part = nullptr;
+    p.z_grid = xcd_grid_size(p.tiles_m * p.tiles_t);
+    p.c_blocks = 0;
     z_ranges(d, p.tiles_m * p.tiles_t, p.ranges, p.range_stages);
     return true;
 }
@@ -459,6 +489,16 @@ static bool spread_ranges(ZParams &p, void *state, void *y, int64_t ldy, const r
     return true;
 }
 
+// The projecting blocks are z_grid: the compute units that they leave free transpose C, where that is a quarter of them at least and the
+// projecting waves would have more than the one unit whose loads their tile's main loop hides (4096 tokens x 1024 -> 1024, k = 64, half a
+// unit a wave: 17.7 us theirs, 17.4 in blocks of its own).
+static void set_z_grid(ZParams &p, int z_grid, int num_cus)
+{
+    p.z_grid = z_grid;
+    const int units = (p.kpad >> 5) * (p.out64 >> 4), spare = (num_cus - z_grid) / 8 * 8;
+    p.c_blocks = p.coef && spare * 4 >= num_cus && units > z_grid * (KZ_THREADS / 64) ? std::min(spare, (int)(cdiv(units, 2 * KZ_THREADS / 64 * 8) * 8)) : 0;
+}
+
 static size_t z_smem() { return engine_smem<KZ_BM, KZ_BT, F_BK, K_CONT, K_CONT>(); }
 
 // y: NULL, or the rows of the forward product to come, free to hold sums on the way
@@ -472,7 +512,8 @@ static int launch_z(void *state, const void *x, int64_t ldx, const void *coef, v
     const size_t smem = z_smem();
     const void *fn = p.ranges > 1 ? (const void *)factored_z_kernel<true> : (const void *)factored_z_kernel<false>;
     if (int rl = reserve_lds(fn, smem, "factored_z_kernel")) return rl;
-    const unsigned grid = xcd_grid_size(p.tiles_m * p.tiles_t) * (spread ? p.ranges : 1);
+    set_z_grid(p, xcd_grid_size(p.tiles_m * p.tiles_t) * (spread ? p.ranges : 1), num_compute_units());
+    const unsigned grid = p.z_grid + p.c_blocks;
     if (p.ranges > 1) factored_z_kernel<true><<<grid, KZ_THREADS, smem, s>>>(p);
     else factored_z_kernel<false><<<grid, KZ_THREADS, smem, s>>>(p);
     return check_launch("factored_z_kernel");
@@ -517,7 +558,7 @@ template <int KG, bool BIAS> static int launch_zy(const ZYParams &p, int y_items
 {
     const size_t smem = std::max(z_smem(), stationary_smem(KG));
     if (int rl = reserve_lds(reinterpret_cast<const void *>(factored_zy_kernel<KG, BIAS>), smem, "factored_zy_kernel")) return rl;
-    factored_zy_kernel<KG, BIAS><<<p.z_blocks + xcd_grid_size(y_items), ST_THREADS, smem, s>>>(p);
+    factored_zy_kernel<KG, BIAS><<<p.z.z_grid + p.z.c_blocks + xcd_grid_size(y_items), ST_THREADS, smem, s>>>(p);
     return check_launch("factored_zy_kernel");
 }
 
@@ -548,7 +589,7 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
     int rc;
     const bool spread = spread_ranges(p.z, state, y, ldy, d, &rc);
     if (rc) return rc;
-    p.z_blocks = xcd_grid_size(p.z.tiles_m * p.z.tiles_t) * (spread ? p.z.ranges : 1);
+    set_z_grid(p.z, xcd_grid_size(p.z.tiles_m * p.z.tiles_t) * (spread ? p.z.ranges : 1), num_cus);
     const int kg = (int)cdiv(d->k, 64);
     if (bias) {
         switch (kg) {

@@ -96,3 +96,28 @@ def test_split_dy_product(T, in_f, out_f, k, with_ct):
     want = (dy.double().cpu() @ c.double().cpu()) @ N.t()
     assert float((out[0][0].double().cpu() - want).norm() / want.norm()) < 8e-3
     assert float((out[0][1].double().cpu() - dy.double().cpu().t() @ (x.double().cpu() @ N)).norm() / (dy.double().cpu().t() @ (x.double().cpu() @ N)).norm()) < 8e-3
+
+
+@pytest.mark.parametrize("T,in_f,out_f,k", [(40, 64, 8, 8), (300, 264, 2056, 72), (1178, 136, 6520, 160), (65, 3080, 40, 256), (300, 1032, 2008, 328)])
+@pytest.mark.parametrize("one_launch", [True, False])
+def test_transposed_coefficients_from_blocks_of_their_own(T, in_f, out_f, k, one_launch):
+    """Few projecting blocks: C is transposed beside them.  The input gradient from the state's transposed coefficients and from C itself:
+    the same bits, from the call that forms y too and from the projection alone."""
+    from randumb_amd import hip
+
+    g = torch.Generator().manual_seed(T)
+    x, dy = torch.randn(T, in_f, generator=g).bfloat16().cuda(), torch.randn(T, out_f, generator=g).bfloat16().cuda()
+    c = (torch.randn(out_f, k, generator=g) / k ** 0.5).bfloat16().cuda()
+    plain = hip.linear_project(x, k, out_f, 5)
+    old = hip.set_one_launch(1 if one_launch else 0)
+    try:
+        y, state = hip.linear_project_fwd(x, c, 5)
+        alone = hip.linear_project(x, k, out_f, 5, coef=c)
+        results = [hip.linear_bwd_projected(dy, s, c, in_f, 5) for s in (state, alone, plain)]
+        hip.sync_check()
+    finally:
+        hip.set_one_launch(old)
+    assert [int(s.view(-1)[:4].view(torch.int32)[0]) for s in (state, alone, plain)] == [1, 1, 0]
+    assert torch.equal(y, hip.linear_fwd_projected(plain, c, in_f, 5))
+    for dx, dc in results[:2]:
+        assert torch.equal(dx, results[2][0]) and torch.equal(dc, results[2][1])

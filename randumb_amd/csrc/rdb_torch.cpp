@@ -15,6 +15,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <atomic>
+#include <initializer_list>
 #include <optional>
 
 #include "../../include/randumb_hip.h"
@@ -45,6 +46,39 @@ void check(int rc, const char *what)
     if (rc == 0) return;
     fail(g_error_class ? g_error_class : PyExc_RuntimeError,
          std::string(what) + ": " + (rc < 0 ? "argument error " : "HIP error ") + std::to_string(rc) + ": " + rdb_last_error_string());
+}
+
+// The library takes raw pointers and looks at none of them: everything a call reads has to lie on the device it runs on.  Called
+// with all tensor arguments before the first launch.
+void same_device(const char *who, const Tensor &at, std::initializer_list<const Tensor *> others)
+{
+    auto check_one = [&](const Tensor &t) {
+        if (!t.is_cuda()) fail(PyExc_NotImplementedError, std::string("Unsupported CPU implementation of ") + who + " called.");
+        if (t.device() != at.device())
+            fail(PyExc_RuntimeError, std::string(who) + ": expected all tensors on " + at.device().str() + ", found one on " + t.device().str());
+    };
+    check_one(at);
+    for (const Tensor *t : others)
+        if (t && t->defined()) check_one(*t);
+}
+const Tensor *address(const OptTensor &t) { return t ? &*t : nullptr; }
+// What a backward pass gets back of a tensor that it saved.  Saved-tensor hooks put in between may return anything: it is used only
+// if it lies on the gradient's device and is what was saved, as far as the kernels rely on it.
+const Tensor &restored(const char *who, const Tensor &t, const Tensor &grad, at::IntArrayRef sizes)
+{
+    if (!t.defined()) fail(PyExc_RuntimeError, std::string(who) + ": a saved tensor is missing");
+    same_device(who, grad, {&t});
+    if (t.sizes() != sizes) fail(PyExc_RuntimeError, std::string(who) + ": a saved tensor came back with another shape");
+    return t;
+}
+// ... of `numel` values (at least) that are read by address
+const Tensor &restored_values(const char *who, const Tensor &t, const Tensor &grad, at::ScalarType type, int64_t numel)
+{
+    if (!t.defined()) fail(PyExc_RuntimeError, std::string(who) + ": a saved tensor is missing");
+    same_device(who, grad, {&t});
+    if (t.scalar_type() != type || !t.is_contiguous() || t.numel() < numel || numel < 0)
+        fail(PyExc_RuntimeError, std::string(who) + ": a saved tensor came back as something else");
+    return t;
 }
 
 void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
@@ -263,6 +297,7 @@ class OneCallLinear : public Function<OneCallLinear> {
         const Bias b{bias, bias_scale, bias_seed};
         ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, l.sO, l.sI, (int64_t)l.seed, scale_bias ? 1 : 0};
         ctx->saved_data["bias"] = b.meta();
+        ctx->saved_data["coefs"] = coefs.sizes().vec();
         const Tensor x = act(x0);
         const bool same = x.scalar_type() == coefs.scalar_type() && readable(coefs.scalar_type()) && (!scale_bias || scale_bias->numel() == 1);
         const rdb_linear_desc d = desc(x, l, coefs);
@@ -286,6 +321,10 @@ class OneCallLinear : public Function<OneCallLinear> {
         const auto m = ctx->saved_data["layer"].toIntVector();
         const Layer l{m[0], m[1], m[2], m[3], (uint32_t)m[4]};
         const bool has_sb = m[5] != 0;
+        constexpr const char *who = "linear (backward)";
+        restored(who, coefs, grads[0], ctx->saved_data["coefs"].toIntVector());
+        if (x.defined()) restored(who, x, grads[0], {grads[0].size(0), l.in_f});
+        if (has_sb) restored(who, sb, grads[0], sb.sizes());
         const at::AutoGradMode no_grad(false);
         const bool want_dx = ctx->needs_input_grad(0), want_dc = ctx->needs_input_grad(1);
         bool want_sb = has_sb && ctx->needs_input_grad(2);
@@ -296,6 +335,8 @@ class OneCallLinear : public Function<OneCallLinear> {
                 const c10::OptionalDeviceGuard guard(dy.device());
                 const Tensor c = coefs.contiguous(), xs = want_sb ? act(x) : Tensor(), s = has_sb ? sb.to(c.scalar_type()) : Tensor();
                 const rdb_linear_desc d = desc(dy, l, c);
+                const int64_t kept_bytes = rdb_linear_kept_bytes(&d);   // 0: the coefficients came back in another dtype
+                restored_values(who, kept, dy, at::kByte, kept_bytes ? kept_bytes : -1);
                 if (want_dx) dx = at::empty({dy.size(0), l.in_f}, dy.options());
                 if (want_dc) dc = at::empty({c.size(0), c.size(1)}, c.options());
                 if (want_sb) dsb = at::empty({1}, dy.options().dtype(at::kFloat));
@@ -364,7 +405,7 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         }
         tick(x);
         ctx->save_for_backward({state, coefs, scale_bias.value_or(Tensor()), scale_bias ? x0 : Tensor()});
-        ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, (int64_t)l.seed, scale_bias ? 1 : 0, pb.tensors()};
+        ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, (int64_t)l.seed, scale_bias ? 1 : 0, pb.tensors(), coefs.size(1)};
         ctx->saved_data["bias"] = pb.meta();
         return y;
     }
@@ -375,6 +416,12 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         const auto m = ctx->saved_data["layer"].toIntVector();
         const Layer l{m[0], m[1], m[0], 1, (uint32_t)m[2]};
         const bool has_sb = m[3] != 0;
+        constexpr const char *who = "linear (backward)";
+        restored(who, coefs, grads[0], {l.out_f, m[5]});
+        if (has_sb) {
+            restored(who, scale_bias, grads[0], scale_bias.sizes());
+            restored(who, saved[3], grads[0], {grads[0].size(0), l.in_f});
+        }
         const at::AutoGradMode no_grad(false);
         const bool want_x = ctx->needs_input_grad(0), want_dc = ctx->needs_input_grad(1), want_sb = has_sb && ctx->needs_input_grad(2 + m[4]);
         const bool want_dx = want_x || want_sb;   // the gradient of the scale comes out of the random-bias share of dx
@@ -384,6 +431,8 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         const Tensor c = coefs.contiguous();
         const c10::OptionalDeviceGuard guard(dy.device());
         const rdb_linear_desc d = desc(dy, l, c);
+        if (c.scalar_type() != dy.scalar_type()) fail(PyExc_RuntimeError, std::string(who) + ": the saved coefficients came back in another dtype");
+        restored_values(who, state, dy, at::kByte, rdb_linear_projection_bytes(&d));
         void *s = stream_of(dy);
         Tensor dx, dc, dsb;
         if (want_dc && (want_dx || f32)) {
@@ -500,8 +549,9 @@ class VectorLinear : public Function<VectorLinear> {
         const bool keep = ctx != nullptr && W.numel() <= x0.numel() + y.numel();
         if (ctx) {
             ctx->save_for_backward({x0, coef, scale.value_or(Tensor()), keep && x0.requires_grad() ? W : Tensor()});
-            ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, (int64_t)l.seed, scale ? (int64_t)scale->scalar_type() : -1};
+            ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, (int64_t)l.seed, scale ? (int64_t)scale->scalar_type() : -1, coef.numel()};
             ctx->saved_data["bias"] = b.meta();
+            ctx->saved_data["x"] = x0.sizes().vec();
         }
         return y;
     }
@@ -520,6 +570,10 @@ class VectorLinear : public Function<VectorLinear> {
         const bool want_x = ctx->needs_input_grad(0), want_c = ctx->needs_input_grad(1), want_s = has_scale && ctx->needs_input_grad(2);
         const Tensor &x0 = saved[0], &coef = saved[1];
         const OptTensor scale = has_scale ? OptTensor(saved[2]) : OptTensor();
+        constexpr const char *who = "linear (backward)";
+        restored(who, x0, grads[0], ctx->saved_data["x"].toIntVector());
+        restored(who, coef, grads[0], {m[4]});
+        if (has_scale) restored(who, saved[2], grads[0], saved[2].sizes());
         const c10::OptionalDeviceGuard guard(x0.device());
         Tensor dx, dc, ds;
         const Tensor dy = act(grads[0].reshape({-1, l.out_f}));
@@ -539,7 +593,9 @@ class VectorLinear : public Function<VectorLinear> {
             return {dx, dc, ds, g[0].to((at::ScalarType)bm[2]), bm[3] >= 0 ? g[1].to((at::ScalarType)bm[3]) : Tensor(), Tensor(), Tensor()};
         }
         if (want_x) {
-            const Tensor W = saved[3].defined() ? saved[3] : coef_values(coef, scale, l.out_f * l.in_f, l.seed).view({l.out_f, l.in_f});
+            const bool kept = saved[3].defined();
+            if (kept) restored(who, restored_values(who, saved[3], dy, x0.scalar_type(), l.out_f * l.in_f), dy, {l.out_f, l.in_f});
+            const Tensor W = kept ? saved[3] : coef_values(coef, scale, l.out_f * l.in_f, l.seed).view({l.out_f, l.in_f});
             dx = product(dy, false, W, true, Tensor()).view(x0.sizes());
         }
         if (want_c || want_s) {
@@ -582,6 +638,7 @@ class EmbedRows : public Function<EmbedRows> {
         const auto m = ctx->saved_data["m"].toIntVector();
         const at::AutoGradMode no_grad(false);
         const Tensor d = native(grads[0]);
+        restored_values("embedding (backward)", idx, d, at::kLong, m[1] ? d.numel() / m[1] : 0);
         const c10::OptionalDeviceGuard guard(d.device());
         Tensor dc = at::empty({m[0]}, d.options().dtype(at::kFloat));
         const int64_t need = rdb_embed_bwd_workspace_bytes(idx.numel(), m[1], m[0]);
@@ -619,6 +676,8 @@ class RmsNorm : public Function<RmsNorm> {
         const auto saved = ctx->get_saved_variables();
         const at::AutoGradMode no_grad(false);
         const Tensor &x = saved[0], dy = grads[0].contiguous();
+        restored_values("rms_norm (backward)", x, dy, at::kBFloat16, dy.numel());
+        restored_values("rms_norm (backward)", saved[1], dy, at::kFloat, row_count(dy));
         const c10::OptionalDeviceGuard guard(x.device());
         Tensor dx = at::empty_like(x);
         check(rdb_rms_norm_bwd(dx.data_ptr(), dy.data_ptr(), x.data_ptr(), nullptr, saved[1].data_ptr<float>(), row_count(x), x.size(-1), stream_of(x)),
@@ -648,6 +707,8 @@ class AddRmsNorm : public Function<AddRmsNorm> {
         const at::AutoGradMode no_grad(false);
         if (!grads[1].defined()) return {grads[0], grads[0], Tensor()};
         const Tensor &x = saved[0], dy = grads[1].contiguous(), dsum = grads[0].defined() ? grads[0].contiguous() : Tensor();
+        restored_values("add_rms_norm (backward)", x, dy, at::kBFloat16, dy.numel());
+        restored_values("add_rms_norm (backward)", saved[1], dy, at::kFloat, row_count(dy));
         const c10::OptionalDeviceGuard guard(x.device());
         Tensor dx = at::empty_like(x);
         check(rdb_rms_norm_bwd(dx.data_ptr(), dy.data_ptr(), x.data_ptr(), ptr(dsum), saved[1].data_ptr<float>(), row_count(x), x.size(-1), stream_of(x)),
@@ -672,6 +733,7 @@ class ReluSquare : public Function<ReluSquare> {
         const Tensor x = ctx->get_saved_variables()[0];
         const at::AutoGradMode no_grad(false);
         const Tensor dy = grads[0].contiguous();
+        restored_values("relu_square (backward)", x, dy, at::kBFloat16, dy.numel());
         const c10::OptionalDeviceGuard guard(x.device());
         Tensor dx = at::empty_like(x);
         check(rdb_relu_square(dx.data_ptr(), x.data_ptr(), dy.data_ptr(), x.numel(), stream_of(x)), "rdb_relu_square");
@@ -692,7 +754,7 @@ class CrossEntropy : public Function<CrossEntropy> {
                                     stream_of(logits)),
               "rdb_cross_entropy_fwd");
         ctx->save_for_backward({logits, target, scratch});
-        ctx->saved_data["ignore"] = ignore;
+        ctx->saved_data["m"] = std::vector<int64_t>{rows, logits.size(1), ignore};
         return loss;
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
@@ -700,10 +762,15 @@ class CrossEntropy : public Function<CrossEntropy> {
         const auto saved = ctx->get_saved_variables();
         const at::AutoGradMode no_grad(false);
         const Tensor &logits = saved[0], dloss = grads[0].to(at::kFloat).contiguous();
+        const auto m = ctx->saved_data["m"].toIntVector();   // rows, classes, ignored label
+        constexpr const char *who = "cross_entropy (backward)";
+        restored(who, restored_values(who, logits, dloss, at::kBFloat16, m[0] * m[1]), dloss, {m[0], m[1]});
+        restored_values(who, saved[1], dloss, at::kLong, m[0]);
+        restored_values(who, saved[2], dloss, at::kFloat, 2 * m[0] + 1);
         const c10::OptionalDeviceGuard guard(logits.device());
         Tensor d = at::empty_like(logits);
         check(rdb_cross_entropy_bwd(d.data_ptr(), logits.data_ptr(), saved[1].data_ptr<int64_t>(), saved[2].data_ptr<float>(), dloss.data_ptr<float>(),
-                                    logits.size(0), logits.size(1), ctx->saved_data["ignore"].toInt(), stream_of(logits)),
+                                    m[0], m[1], m[2], stream_of(logits)),
               "rdb_cross_entropy_bwd");
         return {d, Tensor(), Tensor()};
     }
@@ -732,10 +799,15 @@ class CausalAttention : public Function<CausalAttention> {
         const auto saved = ctx->get_saved_variables();
         const at::AutoGradMode no_grad(false);
         const Tensor &qkv = saved[0], dy = grads[0].contiguous();
+        constexpr const char *who = "causal_attention (backward)";
+        const int64_t B = dy.size(0), T = dy.size(1), heads = ctx->saved_data["heads"].toInt();
+        restored(who, restored_values(who, qkv, dy, at::kBFloat16, 3 * dy.numel()), dy, {B, T, 3 * heads * 64});
+        for (int i = 1; i < 4; ++i) restored_values(who, saved[i], dy, at::kBFloat16, dy.numel());
+        restored_values(who, saved[4], dy, at::kFloat, rdb_causal_attention_scratch_floats(B, T, heads));
         const c10::OptionalDeviceGuard guard(qkv.device());
         Tensor d = at::empty_like(qkv);
         check(rdb_causal_attention_bwd(d.data_ptr(), dy.data_ptr(), saved[1].data_ptr(), saved[2].data_ptr(), saved[3].data_ptr(), saved[4].data_ptr<float>(),
-                                       qkv.data_ptr(), qkv.size(0), qkv.size(1), ctx->saved_data["heads"].toInt(), (float)ctx->saved_data["eps"].toDouble(),
+                                       qkv.data_ptr(), B, T, heads, (float)ctx->saved_data["eps"].toDouble(),
                                        stream_of(qkv)),
               "rdb_causal_attention_bwd");
         return {d, Tensor(), Tensor(), Tensor()};
@@ -832,6 +904,7 @@ PyObject *py_linear_projected(PyObject *, PyObject *const *a, Py_ssize_t n)
         const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[2]), 1, seed_arg(a[4])};
         const Bias b = bias_arg(a + 5);
         const OptTensor sb = opt_arg(a[8]);
+        same_device("linear_fwd", x, {&c, address(b.coef), address(b.scale), address(sb)});
         // without a backward pass to come there is no state to keep: the one-call forward
         if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
             return THPVariable_Wrap(linear_fwd(x, c, l, sb, b));
@@ -848,6 +921,7 @@ PyObject *py_linear_one_call(PyObject *, PyObject *const *a, Py_ssize_t n)
         const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[4]), int_arg(a[5]), seed_arg(a[6])};
         const OptTensor sb = opt_arg(a[7]);
         const Bias b = bias_arg(a + 8);
+        same_device("linear_fwd", x, {&c, address(b.coef), address(b.scale), address(sb)});
         if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
             return THPVariable_Wrap(linear_fwd(x, c, l, sb, b));
         return THPVariable_Wrap(OneCallLinear::apply(x, c, sb, b.coef, b.scale, b.seed, l));
@@ -863,6 +937,7 @@ PyObject *py_linear_vector(PyObject *, PyObject *const *a, Py_ssize_t n)
         const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[2]), 1, seed_arg(a[4])};
         const OptTensor sb = opt_arg(a[5]);
         const Bias b = bias_arg(a + 6);
+        same_device("linear_vector", x, {&c, address(b.coef), address(b.scale), address(sb)});
         if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
             return THPVariable_Wrap(VectorLinear::forward(nullptr, x, c, sb, b.coef, b.scale, b.seed, l));
         return THPVariable_Wrap(VectorLinear::apply(x, c, sb, b.coef, b.scale, b.seed, l));
@@ -876,6 +951,7 @@ PyObject *py_embed_rows(PyObject *, PyObject *const *a, Py_ssize_t n)
         count_args(n, 4);
         const Tensor &idx = tensor_arg(a[0]), &c = tensor_arg(a[1]);
         const int64_t rowsize = int_arg(a[2]), seed = seed_arg(a[3]);
+        same_device("embed_fwd", idx, {&c});
         if (!at::GradMode::is_enabled() || !c.requires_grad()) return THPVariable_Wrap(EmbedRows::forward(nullptr, idx, c, rowsize, seed));
         return THPVariable_Wrap(EmbedRows::apply(idx, c, rowsize, seed));
     });
@@ -907,6 +983,7 @@ PyObject *py_add_rms_norm(PyObject *, PyObject *const *a, Py_ssize_t n)
         const Tensor &x = tensor_arg(a[0]), &delta = tensor_arg(a[1]);
         need_bf16("add_rms_norm", x);
         need_bf16("add_rms_norm", delta);
+        same_device("add_rms_norm", x, {&delta});
         if (x.sizes() != delta.sizes()) fail(PyExc_ValueError, "add_rms_norm needs tensors of one shape");
         const auto r = AddRmsNorm::apply(x, delta, float_arg(a[2]));
         PyObject *s = THPVariable_Wrap(r[0]), *y = THPVariable_Wrap(r[1]);

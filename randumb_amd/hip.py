@@ -18,9 +18,16 @@ _DT = {torch.float32: RDB_F32, torch.bfloat16: RDB_BF16}
 
 
 def _need_gpu(name: str, *tensors) -> None:
+    """All tensors of a call on one GPU: the library takes raw pointers and looks at none of them."""
+    at = None
     for t in tensors:
-        if t is not None and not t.is_cuda:
+        if t is None:
+            continue
+        if not t.is_cuda:
             raise NotImplementedError(f"Unsupported CPU implementation of {name} called.")
+        at = t.device if at is None else at
+        if t.device != at:
+            raise RuntimeError(f"{name}: expected all tensors on {at}, found one on {t.device}")
 
 
 def _native(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
@@ -202,7 +209,7 @@ def materialize_fwd(coefs: torch.Tensor, size: Sequence[int], strides: Sequence[
     (RandumbTensor.py:371-381).  ``coefs.dim() == 2`` selects the matrix-coef form, whose base tensor is
     ``(coefs.shape[0], row_len)`` contiguous (``row_len`` defaults to ``numel / coefs.shape[0]``)."""
     assert not (fused_bias and scale_bias is None), "scale_bias not initialized but fused_bias is True"
-    _need_gpu("materialize_fwd", coefs)
+    _need_gpu("materialize_fwd", coefs, scale_bias if fused_bias else None)
     size, strides = [int(s) for s in size], [int(s) for s in strides]
     output = torch.empty(size, dtype=torch.float32, device=coefs.device)
     if len(size) == 1:  # RandumbTensor.py:375-377
@@ -322,7 +329,7 @@ def linear_fwd(x: torch.Tensor, coef: torch.Tensor, in_f: int, out_f: int, sO: i
                scale_bias: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None,
                algo: int = RDB_ALGO_AUTO) -> torch.Tensor:
     """``y = x @ W.T (+ bias)`` with the ``(out_f, in_f)`` pseudorandom weight regenerated on chip."""
-    _need_gpu("linear_fwd", x, coef)
+    _need_gpu("linear_fwd", x, coef, scale_bias, bias)
     x = _act(x)
     c = _native(coef)
     sb = None if scale_bias is None else _native(scale_bias).to(c.dtype)
@@ -343,7 +350,7 @@ def linear_fwd(x: torch.Tensor, coef: torch.Tensor, in_f: int, out_f: int, sO: i
 def linear_bwd_dx(dy: torch.Tensor, coef: torch.Tensor, in_f: int, out_f: int, sO: int, sI: int, seed: int,
                   scale_bias: Optional[torch.Tensor] = None, algo: int = RDB_ALGO_AUTO) -> torch.Tensor:
     """``dx = dy @ W``."""
-    _need_gpu("linear_bwd_dx", dy, coef)
+    _need_gpu("linear_bwd_dx", dy, coef, scale_bias)
     dy = _act(dy)
     c = _native(coef)
     sb = None if scale_bias is None else _native(scale_bias).to(c.dtype)
@@ -418,7 +425,7 @@ def linear_rbias_bwd_(dx: torch.Tensor, dy: torch.Tensor, x: Optional[torch.Tens
                       seed: int, want_scale_bias_grad: bool = False) -> Optional[torch.Tensor]:
     """In place: ``dx += scale_bias * dy @ R``; returns the gradient of the scale, ``<dy @ R, x>`` (fp32, ``(1,)``), from the same
     pass when asked for (``x`` is needed then only)."""
-    _need_gpu("linear_rbias_bwd_", dx, dy, scale_bias)
+    _need_gpu("linear_rbias_bwd_", dx, dy, scale_bias, x if want_scale_bias_grad else None)
     dy = _act(dy)
     sb = _native(scale_bias).to(torch.bfloat16)
     d = _rbias_desc(dy.shape[0], in_f, out_f, seed)
@@ -574,8 +581,7 @@ def linear_project(x: torch.Tensor, k: int, out_f: int, seed: int, coef: Optiona
 def linear_project_fwd(x: torch.Tensor, coef: torch.Tensor, seed: int, bias: Optional[torch.Tensor] = None):
     """``(y, state)``: :func:`linear_project` (with ``coef``) and :func:`linear_fwd_projected` in one call, for k <= 256 in a
     single kernel launch; the forward pass of a training step, ``state`` being what it saves for backward."""
-    if not (x.is_cuda and coef.is_cuda):
-        _need_gpu("linear_project_fwd", x, coef)
+    _need_gpu("linear_project_fwd", x, coef, bias)
     x = _act(x)
     c = coef if coef.is_contiguous() else coef.contiguous()
     if x.dtype != c.dtype or x.dtype not in _DT:
@@ -648,7 +654,7 @@ def linear_fwd_projected(state: torch.Tensor, coef: torch.Tensor, in_f: int, see
                          bias: Optional[torch.Tensor] = None, f32_state: bool = False) -> torch.Tensor:
     """``y = z @ coef.T (+ bias)`` for matrix-coef ``coef`` (out_f, k) in bf16; ``state`` from :func:`linear_project`.
     ``f32_state``: the state is that of an fp32 layer (fp32 activations and coefficients)."""
-    _need_gpu("linear_fwd_projected", state, coef)
+    _need_gpu("linear_fwd_projected", state, coef, bias)
     c = _native(coef)
     out_f, k = c.shape
     tokens = state.shape[0]
@@ -703,8 +709,7 @@ def linear_bwd_projected(dy: torch.Tensor, state: torch.Tensor, coef: torch.Tens
     ``.to(bfloat16)`` would give, without the extra pass; layers whose tokens the library runs in several chunks get fp32 sums
     rounded by torch instead).  fp32 layers (``dy`` and ``coef`` in fp32): sums in fp32 in a fixed order; ``want_dx=False``
     returns ``(None, dcoef)``."""
-    if not (dy.is_cuda and state.is_cuda and coef.is_cuda):
-        _need_gpu("linear_bwd_projected", dy, state, coef)
+    _need_gpu("linear_bwd_projected", dy, state, coef)
     dy = _act(dy)
     c = _native(coef)
     out_f, k = c.shape

@@ -1,0 +1,81 @@
+"""What is refused, and what goes on working, around the calls that reach kernels by address."""
+import pytest
+import torch
+
+from randumb_amd import SillyEmbedding, SillyLinear, _lib, listgen
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(form):
+    """(layer, input) of every way a layer's forward pass saves for its backward pass."""
+    dt = torch.float32 if form.endswith("fp32") else torch.bfloat16
+    sizes = {"projected_bf16": (300, 256, 192, 64), "projected_fp32": (300, 256, 192, 128), "random_bias_bf16": (300, 256, 192, 64),
+             "kept_bf16": (130, 133, 99, 50), "one_call_fp32": (3, 256, 192, 16), "vector_fp32": (40, 96, 64, 16)}
+    tokens, in_f, out_f, k = sizes[form]
+    layer = SillyLinear(in_f, out_f, [k, k], [1, 2], device="cuda", dtype=dt, matrix_coef=not form.startswith("vector"), rt_bias=form.startswith("random"))
+    with torch.no_grad():
+        for p in (layer.weight_coef, layer.bias_coef):
+            p.normal_(0.0, 0.05)
+    return layer, torch.randn(tokens, in_f, device="cuda").to(dt).requires_grad_()
+
+
+FORMS = ["projected_bf16", "projected_fp32", "random_bias_bf16", "kept_bf16", "one_call_fp32", "vector_fp32"]
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_saved_tensors_that_come_back_on_the_host_are_refused(form):
+    """Hooks that pack saved tensors to the host and do not bring them back: an exception from the backward pass."""
+    layer, x = _layer(form)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t):
+        y = layer(x)
+    with pytest.raises(NotImplementedError, match="CPU implementation"):
+        y.backward(torch.ones_like(y))
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_saved_tensors_may_rest_on_the_host(form):
+    layer, x = _layer(form)
+    wanted = [x, *layer.parameters()]
+    y = layer(x)
+    ref = torch.autograd.grad(y, wanted, torch.ones_like(y), allow_unused=True)
+    with torch.autograd.graph.save_on_cpu():
+        y = layer(x)
+    got = torch.autograd.grad(y, wanted, torch.ones_like(y), allow_unused=True)
+    for a, b in zip(got, ref):
+        assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+
+
+def test_saved_indices_of_the_embedding_on_the_host_are_refused():
+    e = SillyEmbedding(50, 24, listgen([16]), listgen([3]), device="cuda")
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t):
+        y = e(torch.tensor([1, 5, 49], device="cuda"))
+    with pytest.raises(NotImplementedError, match="CPU implementation"):
+        y.sum().backward()
+
+
+@pytest.mark.parametrize("op", ["rms_norm", "add_rms_norm", "relu_square", "cross_entropy", "causal_attention"])
+def test_saved_activations_on_the_host_are_refused(op):
+    ext = _lib.extension()
+    x = torch.randn(2, 8, 3 * 64, device="cuda").bfloat16().requires_grad_()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t):
+        if op == "rms_norm":
+            y = ext.rms_norm(x, 1e-6)
+        elif op == "add_rms_norm":
+            y = ext.add_rms_norm(x, x.detach(), 1e-6)[1]
+        elif op == "relu_square":
+            y = ext.relu_square(x)
+        elif op == "cross_entropy":
+            y = ext.cross_entropy(x.view(-1, 192), torch.zeros(16, dtype=torch.int64, device="cuda"), -100)
+        else:
+            y = ext.causal_attention(x, torch.ones(32, device="cuda"), 1, 1e-6)
+    with pytest.raises(NotImplementedError, match="CPU implementation"):
+        y.backward(torch.ones_like(y))
+
+
+def test_a_layer_and_an_input_on_different_devices_are_refused():
+    layer = SillyLinear(768, 96, [32, 32], [1, 2], matrix_coef=True)
+    with pytest.raises(NotImplementedError, match="CPU implementation"):
+        layer(torch.randn(4, 768, device="cuda"))
+    layer = layer.to("cuda")
+    assert layer(torch.randn(4, 768, device="cuda")).shape == (4, 96)

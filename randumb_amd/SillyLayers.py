@@ -170,6 +170,8 @@ class SillyLinear(SillyModuleMixin, nn.Module):
         in_f, out_f = self.in_features, self.out_features
         w = self._buffers["weight"]   # past nn.Module's attribute search: a few-token layer's kernels take less than a forward's host time
         flat = input.dim() == 2
+        if input.dim() > 1 and input.shape[-1] != in_f:
+            raise RuntimeError(f"a layer {in_f} -> {out_f} cannot take an input of shape {tuple(input.shape)}")
         x2 = input if flat else input.reshape(-1, in_f)
         if x2.dtype != w.dtype:
             x2 = x2.to(w.dtype)

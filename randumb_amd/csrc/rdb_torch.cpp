@@ -814,6 +814,22 @@ class CausalAttention : public Function<CausalAttention> {
     }
 };
 
+// The sizes the descriptor states are those of the tensors: the library is told in_f and out_f and reads that far.
+void check_sizes(const char *who, const Tensor &x, const Tensor &c, const Layer &l, const OptTensor &scale, const Bias &b)
+{
+    auto wrong = [&](const char *what, const Tensor &t) {
+        std::string sizes;
+        for (int64_t n : t.sizes()) sizes += (sizes.empty() ? "" : ", ") + std::to_string(n);
+        fail(PyExc_RuntimeError, std::string(who) + ": a layer " + std::to_string(l.in_f) + " -> " + std::to_string(l.out_f) + " cannot take " + what + " of shape (" +
+                                     sizes + ")");
+    };
+    if (x.dim() < 1 || x.size(-1) != l.in_f) wrong("an input", x);
+    if (c.dim() != 1 && c.dim() != 2) wrong("coefficients", c);
+    if (scale && scale->numel() < 1) wrong("a scale", *scale);
+    if (b.coef && (b.seed < 0 ? b.coef->numel() != l.out_f : b.coef->dim() != 1)) wrong(b.seed < 0 ? "a bias" : "bias coefficients", *b.coef);
+    if (b.scale && b.scale->numel() < 1) wrong("a bias scale", *b.scale);
+}
+
 // ----------------------------------------------------------------------------------------------- Python methods
 struct BadArgument {};
 
@@ -905,6 +921,7 @@ PyObject *py_linear_projected(PyObject *, PyObject *const *a, Py_ssize_t n)
         const Bias b = bias_arg(a + 5);
         const OptTensor sb = opt_arg(a[8]);
         same_device("linear_fwd", x, {&c, address(b.coef), address(b.scale), address(sb)});
+        check_sizes("linear_fwd", x, c, l, sb, b);
         // without a backward pass to come there is no state to keep: the one-call forward
         if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
             return THPVariable_Wrap(linear_fwd(x, c, l, sb, b));
@@ -922,6 +939,7 @@ PyObject *py_linear_one_call(PyObject *, PyObject *const *a, Py_ssize_t n)
         const OptTensor sb = opt_arg(a[7]);
         const Bias b = bias_arg(a + 8);
         same_device("linear_fwd", x, {&c, address(b.coef), address(b.scale), address(sb)});
+        check_sizes("linear_fwd", x, c, l, sb, b);
         if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
             return THPVariable_Wrap(linear_fwd(x, c, l, sb, b));
         return THPVariable_Wrap(OneCallLinear::apply(x, c, sb, b.coef, b.scale, b.seed, l));
@@ -938,6 +956,7 @@ PyObject *py_linear_vector(PyObject *, PyObject *const *a, Py_ssize_t n)
         const OptTensor sb = opt_arg(a[5]);
         const Bias b = bias_arg(a + 6);
         same_device("linear_vector", x, {&c, address(b.coef), address(b.scale), address(sb)});
+        check_sizes("linear_vector", x, c, l, sb, b);
         if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
             return THPVariable_Wrap(VectorLinear::forward(nullptr, x, c, sb, b.coef, b.scale, b.seed, l));
         return THPVariable_Wrap(VectorLinear::apply(x, c, sb, b.coef, b.scale, b.seed, l));

@@ -316,6 +316,17 @@ def _desc(tokens, in_f, out_f, coef, sO, sI, seed, act_dtype, algo) -> LinearDes
     return d
 
 
+def _need_shape(name: str, what: str, t: Optional[torch.Tensor], *shape) -> None:
+    """A tensor of the stated sizes (None: any): the library is told the sizes and reads that far."""
+    if t is not None and (t.dim() != len(shape) or any(n is not None and t.shape[i] != n for i, n in enumerate(shape))):
+        raise RuntimeError(f"{name}: {what} must have shape ({', '.join('*' if n is None else str(n) for n in shape)}), got {tuple(t.shape)}")
+
+
+def _need_bias(name: str, bias: Optional[torch.Tensor], out_f: int) -> None:
+    if bias is not None and bias.numel() != out_f:
+        raise RuntimeError(f"{name}: the bias must have {out_f} values, got shape {tuple(bias.shape)}")
+
+
 def _act(t: torch.Tensor) -> torch.Tensor:
     """2-D activation with unit inner stride in a dtype the kernels compute in."""
     if t.dtype not in _DT:
@@ -331,6 +342,8 @@ def linear_fwd(x: torch.Tensor, coef: torch.Tensor, in_f: int, out_f: int, sO: i
     """``y = x @ W.T (+ bias)`` with the ``(out_f, in_f)`` pseudorandom weight regenerated on chip."""
     _need_gpu("linear_fwd", x, coef, scale_bias, bias)
     x = _act(x)
+    _need_shape("linear_fwd", "the input", x, None, in_f)
+    _need_bias("linear_fwd", bias, out_f)
     c = _native(coef)
     sb = None if scale_bias is None else _native(scale_bias).to(c.dtype)
     b = None if bias is None else bias.to(x.dtype).contiguous()
@@ -352,6 +365,7 @@ def linear_bwd_dx(dy: torch.Tensor, coef: torch.Tensor, in_f: int, out_f: int, s
     """``dx = dy @ W``."""
     _need_gpu("linear_bwd_dx", dy, coef, scale_bias)
     dy = _act(dy)
+    _need_shape("linear_bwd_dx", "the gradient", dy, None, out_f)
     c = _native(coef)
     sb = None if scale_bias is None else _native(scale_bias).to(c.dtype)
     dx = torch.empty((dy.shape[0], in_f), dtype=dy.dtype, device=dy.device)
@@ -378,6 +392,8 @@ def linear_bwd_dx_dscale(dy: torch.Tensor, x: torch.Tensor, coef: torch.Tensor, 
     if x.dtype != dy.dtype:
         x = x.to(dy.dtype)
     c = _native(coef)
+    _need_shape("linear_bwd_dx_dscale", "the gradient", dy, None, out_f)
+    _need_shape("linear_bwd_dx_dscale", "the input", x, dy.shape[0], in_f)
     sb = _native(scale_bias).to(c.dtype)
     d = _desc(dy.shape[0], in_f, out_f, c, in_f, 1, seed, dy.dtype, RDB_ALGO_AUTO)
     L = _lib.load()
@@ -413,6 +429,8 @@ def linear_rbias_fwd_(y: torch.Tensor, x: torch.Tensor, scale_bias: torch.Tensor
     ``W = C.N + s.R`` (src/rten_cpp/RandumbTensor.py:286-289), on top of a ``y`` that holds the low-rank share.  bf16."""
     _need_gpu("linear_rbias_fwd_", y, x, scale_bias)
     x = _act(x)
+    _need_shape("linear_rbias_fwd_", "the input", x, None, in_f)
+    _need_shape("linear_rbias_fwd_", "y", y, x.shape[0], out_f)
     sb = _native(scale_bias).to(torch.bfloat16)
     d = _rbias_desc(x.shape[0], in_f, out_f, seed)
     with _on(x.device):
@@ -427,6 +445,9 @@ def linear_rbias_bwd_(dx: torch.Tensor, dy: torch.Tensor, x: Optional[torch.Tens
     pass when asked for (``x`` is needed then only)."""
     _need_gpu("linear_rbias_bwd_", dx, dy, scale_bias, x if want_scale_bias_grad else None)
     dy = _act(dy)
+    _need_shape("linear_rbias_bwd_", "the gradient", dy, None, out_f)
+    _need_shape("linear_rbias_bwd_", "dx", dx, dy.shape[0], in_f)
+    _need_shape("linear_rbias_bwd_", "the input", x if want_scale_bias_grad else None, dy.shape[0], in_f)
     sb = _native(scale_bias).to(torch.bfloat16)
     d = _rbias_desc(dy.shape[0], in_f, out_f, seed)
     L = _lib.load()
@@ -449,6 +470,8 @@ def linear_bwd_dcoef(dy: torch.Tensor, x: torch.Tensor, k: int, coef_rows: int, 
     """``(dcoef, d_scale_bias)`` in fp32: ``dcoef = (dy.T @ x) . Noise.T`` without storing ``dy.T @ x``."""
     _need_gpu("linear_bwd_dcoef", dy, x)
     dy, x = _act(dy), _act(x)
+    _need_shape("linear_bwd_dcoef", "the gradient", dy, None, out_f)
+    _need_shape("linear_bwd_dcoef", "the input", x, dy.shape[0], in_f)
     if x.dtype != dy.dtype:
         x = x.to(dy.dtype)
     shape = (k,) if coef_rows == 0 else (coef_rows, k)
@@ -588,6 +611,7 @@ def linear_project_fwd(x: torch.Tensor, coef: torch.Tensor, seed: int, bias: Opt
         raise ValueError("linear_project_fwd computes in bf16 or in fp32: activations and coefficients in one of them")
     out_f, k = c.shape
     tokens = x.shape[0]
+    _need_bias("linear_project_fwd", bias, out_f)
     pl = _plan(tokens, x.shape[1], out_f, k, seed, x.dtype)
     L = _lib.load()
     if pl.state_bytes <= 0:
@@ -658,6 +682,7 @@ def linear_fwd_projected(state: torch.Tensor, coef: torch.Tensor, in_f: int, see
     c = _native(coef)
     out_f, k = c.shape
     tokens = state.shape[0]
+    _need_bias("linear_fwd_projected", bias, out_f)
     act = torch.float32 if (f32_state and c.dtype == torch.float32) else torch.bfloat16
     d = _proj_desc(tokens, in_f, out_f, k, seed, c.dtype, act)
     _check_state(state, d, "linear_fwd_projected")
@@ -714,6 +739,7 @@ def linear_bwd_projected(dy: torch.Tensor, state: torch.Tensor, coef: torch.Tens
     c = _native(coef)
     out_f, k = c.shape
     tokens = dy.shape[0]
+    _need_shape("linear_bwd_projected", "the gradient", dy, None, out_f)
     f32 = dy.dtype == torch.float32 and c.dtype == torch.float32
     pl = _plan(tokens, in_f, out_f, k, seed, torch.float32 if f32 else torch.bfloat16)
     if not f32 and c.dtype != torch.bfloat16:

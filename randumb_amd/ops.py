@@ -386,11 +386,12 @@ def _coef_form(t) -> Optional[tuple]:
     return c, sb, t.seed
 
 
-def _bias_form(bias) -> Optional[tuple]:
-    """The three arguments the extension module takes for a bias; None where it does not take this one."""
+def _bias_form(bias, out_features: int) -> Optional[tuple]:
+    """The three arguments the extension module takes for a bias; None where it does not take this one (of a pseudorandom bias it
+    only sees the coefficients, so the length is looked at here)."""
     if bias is None or not hasattr(bias, "get_materialized"):
         return bias, None, -1
-    return _coef_form(bias) if bias.dim() == 1 else None
+    return _coef_form(bias) if bias.dim() == 1 and bias.shape[0] == out_features else None
 
 
 class _ProjectedLinear:
@@ -399,7 +400,7 @@ class _ProjectedLinear:
 
     @staticmethod
     def apply(x, coefs, in_features, out_features, seed, bias, scale_bias=None):
-        form = None if _tracing() or hip.CHECK_STATE_COEF else _bias_form(bias)
+        form = None if _tracing() or hip.CHECK_STATE_COEF else _bias_form(bias, out_features)
         if form is None:
             return _ProjectedFunction.apply(x, coefs, in_features, out_features, seed, bias, scale_bias)
         return _lib.extension().linear_projected(x, coefs, in_features, out_features, seed, *form, scale_bias)
@@ -414,7 +415,7 @@ def linear(x: Tensor, coefs: Tensor, in_features: int, out_features: int, stride
         ext = _lib._ext or _lib.extension()
         if ext.takes_projected(x, coefs, in_features, out_features, stride_o, stride_i, scale_bias, bias):
             return _ProjectedLinear.apply(x, coefs, in_features, out_features, seed, bias, scale_bias)
-        form = _bias_form(bias)
+        form = _bias_form(bias, out_features)
         if form is None:
             return _OneCallFunction.apply(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias)
         return ext.linear_one_call(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, *form)
@@ -435,7 +436,9 @@ def vector_linear(x: Tensor, weight, bias) -> Optional[Tensor]:
     if (not x.is_cuda or x.dim() < 2 or type(x) not in (Tensor, torch.nn.Parameter) or x.dtype not in (torch.float32, torch.bfloat16)
             or x.dtype != weight.dtype or weight.dim() != 2 or x.shape[-1] != weight.shape[1] or _tracing() or torch.is_autocast_enabled()):
         return None
-    w, b = _coef_form(weight), _bias_form(bias)
+    if bias is not None and (bias.dtype != x.dtype or bias.shape != (weight.shape[0],)):
+        return None   # F.linear broadcasts the one and refuses the other
+    w, b = _coef_form(weight), _bias_form(bias, weight.shape[0])
     if w is None or b is None or x.device != w[0].device:
         return None
     return (_lib._ext or _lib.extension()).linear_vector(x, w[0], weight.shape[1], weight.shape[0], w[2], w[1], *b)

@@ -9,7 +9,7 @@ from randumb_amd import SillyLinear, _lib, ops
 
 def _fake(*shape, dtype=torch.float32, device="cuda:0"):
     with FakeTensorMode():
-        return torch.empty(*shape, dtype=dtype, device=device)
+        return torch.empty(shape, dtype=dtype, device=device)
 
 
 IN, OUT, K = 768, 96, 32
@@ -61,3 +61,62 @@ def test_the_operators_refuse_a_host_scale_or_bias(name):
     kw = {name: torch.zeros(OUT if name == "bias" else 1)}
     with pytest.raises(NotImplementedError, match="CPU implementation"):
         hip.linear_fwd(_fake(4, IN), _fake(OUT, K), IN, OUT, IN, 1, 3, **kw)
+
+
+# ------------------------------------------------------------------------------------------------ sizes that are the layer's
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("width", [IN + 256, IN - 8, 1])
+def test_an_input_of_another_width_is_refused(width, fused, monkeypatch):
+    """A 2-D input is passed on as it is: wider ones are not cut, narrower ones not read past their rows."""
+    ran = []
+    monkeypatch.setattr(ops, "linear", lambda *a: ran.append(a))
+    layer = SillyLinear(IN, OUT, [K, K], [1, 2], matrix_coef=fused)
+    with pytest.raises((RuntimeError, NotImplementedError)):
+        layer(torch.zeros(4, width))
+    with pytest.raises((RuntimeError, NotImplementedError)):
+        layer(torch.zeros(2, 3, width))
+    assert not ran
+
+
+@pytest.mark.parametrize("entry", ["one_call", "projected", "vector"])
+def test_the_entry_points_refuse_sizes_that_are_not_the_layers(entry):
+    ext = _lib.extension()
+
+    def call(x=(4, IN), coefs=(K,) if entry == "vector" else (OUT, K), scale=(1,), bias=((OUT,), None, -1)):
+        x, c, sb = _fake(*x), _fake(*coefs), _fake(*scale)
+        b = tuple(_fake(*v) if isinstance(v, tuple) else v for v in bias)
+        if entry == "one_call":
+            ext.linear_one_call(x, c, IN, OUT, IN, 1, 3, sb, *b)
+        elif entry == "projected":
+            ext.linear_projected(x, c, IN, OUT, 3, *b, sb)
+        else:
+            ext.linear_vector(x, c, IN, OUT, 3, sb, *b)
+
+    for what, args in (("an input", {"x": (4, IN + 256)}), ("an input", {"x": (4, IN - 8)}), ("an input", {"x": ()}), ("coefficients", {"coefs": (2, OUT, K)}),
+                       ("a scale", {"scale": (0,)}), ("a bias", {"bias": ((1,), None, -1)}), ("a bias", {"bias": ((OUT + 1,), None, -1)}),
+                       ("bias coefficients", {"bias": ((2, K), None, 3)}), ("a bias scale", {"bias": ((K,), (0,), 3)})):
+        with pytest.raises(RuntimeError, match=f"cannot take {what} of shape"):
+            call(**args)
+
+
+def test_the_operators_refuse_sizes_that_are_not_the_layers():
+    from randumb_amd import hip
+
+    x, c, dy = _fake(4, IN), _fake(OUT, K), _fake(4, OUT)
+    one = _fake(1)
+    for call in (lambda: hip.linear_fwd(_fake(4, IN + 8), c, IN, OUT, IN, 1, 3), lambda: hip.linear_fwd(x, c, IN, OUT, IN, 1, 3, bias=_fake(OUT - 1)),
+                 lambda: hip.linear_bwd_dx(_fake(4, OUT - 8), c, IN, OUT, IN, 1, 3),
+                 lambda: hip.linear_bwd_dcoef(dy, _fake(5, IN), K, OUT, IN, OUT, IN, 1, 3), lambda: hip.linear_bwd_dcoef(_fake(4, 8), x, K, OUT, IN, OUT, IN, 1, 3),
+                 lambda: hip.linear_project_fwd(x, c, 3, bias=_fake(OUT + 8)), lambda: hip.linear_rbias_fwd_(_fake(3, OUT), x, one, IN, OUT, 3),
+                 lambda: hip.linear_rbias_bwd_(_fake(4, IN), dy, _fake(4, OUT), one, IN, OUT, 3, want_scale_bias_grad=True),
+                 lambda: hip.linear_bwd_projected(_fake(4, 8), _fake(4, 8), c, IN, 3)):
+        with pytest.raises(RuntimeError, match="must have"):
+            call()
+
+
+def test_a_bias_of_another_length_or_type_is_left_to_the_general_path():
+    """Of a pseudorandom bias the extension module sees coefficients only; a dense one F.linear broadcasts or refuses."""
+    from randumb_amd import CreateRandumbTensor
+
+    bias = CreateRandumbTensor(torch.zeros(K), 1, (OUT,))
+    assert ops._bias_form(bias, OUT) is not None and ops._bias_form(bias, OUT + 1) is None

@@ -168,7 +168,14 @@ class SillyLinear(SillyModuleMixin, nn.Module):
             y = ops.vector_linear(input, w, b) if isinstance(w, RandumbTensor) and not (w.FUSED_MM and w.FUSED_MM_VECTOR) else None
             return F.linear(input, w, b) if y is None else y
         in_f, out_f = self.in_features, self.out_features
-        w = self._buffers["weight"]   # past nn.Module's attribute search: a few-token layer's kernels take less than a forward's host time
+        # where a layer is built its tensors are looked up past nn.Module's attribute search (a few-token layer's kernels take less than a
+        # forward's host time); parametrizations, pruning, replicas and replaced biases put them elsewhere
+        w = self._buffers.get("weight")
+        if w is None:
+            w = self.weight
+        coef = self._parameters.get("weight_coef")
+        if coef is None:
+            coef = self.weight_coef
         flat = input.dim() == 2
         if input.dim() > 1 and input.shape[-1] != in_f:
             raise RuntimeError(f"a layer {in_f} -> {out_f} cannot take an input of shape {tuple(input.shape)}")
@@ -176,8 +183,8 @@ class SillyLinear(SillyModuleMixin, nn.Module):
         if x2.dtype != w.dtype:
             x2 = x2.to(w.dtype)
         sb = w.scale_bias if w.fused_bias else None
-        bias = self._buffers["bias"] if "bias" in self._buffers else None
-        y = ops.linear(x2, self._parameters["weight_coef"], in_f, out_f, in_f, 1, w.seed, sb, bias)
+        bias = self._buffers["bias"] if "bias" in self._buffers else self.bias
+        y = ops.linear(x2, coef, in_f, out_f, in_f, 1, w.seed, sb, bias)
         return y if flat else y.reshape(*input.shape[:-1], out_f)
 
     def extra_repr(self) -> str:

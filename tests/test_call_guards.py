@@ -120,3 +120,62 @@ def test_a_bias_of_another_length_or_type_is_left_to_the_general_path():
 
     bias = CreateRandumbTensor(torch.zeros(K), 1, (OUT,))
     assert ops._bias_form(bias, OUT) is not None and ops._bias_form(bias, OUT + 1) is None
+
+
+# ------------------------------------------------------------------------------------------------ tensors that are not where a layer puts them
+def _what_linear_gets(monkeypatch, layer):
+    got = {}
+
+    def linear(x, coefs, in_f, out_f, sO, sI, seed, scale_bias, bias):
+        got.update(coefs=coefs, bias=bias, seed=seed)
+        return x.new_zeros(x.shape[0], out_f)
+
+    monkeypatch.setattr(ops, "linear", linear)
+    layer(torch.zeros(4, IN))
+    return got
+
+
+def test_a_parametrized_coefficient_is_used(monkeypatch):
+    class Doubled(torch.nn.Module):
+        def forward(self, c):
+            return 2 * c
+
+    layer = SillyLinear(IN, OUT, [K, K], [1, 2], matrix_coef=True)
+    with torch.no_grad():
+        layer.weight_coef.normal_()
+    before = layer.weight_coef.detach().clone()
+    torch.nn.utils.parametrize.register_parametrization(layer, "weight_coef", Doubled())
+    got = _what_linear_gets(monkeypatch, layer)
+    assert torch.equal(got["coefs"], 2 * before) and got["coefs"].requires_grad
+
+
+def test_a_pruned_coefficient_is_used(monkeypatch):
+    from torch.nn.utils import prune
+
+    layer = SillyLinear(IN, OUT, [K, K], [1, 2], matrix_coef=True)
+    with torch.no_grad():
+        layer.weight_coef.normal_()
+    prune.random_unstructured(layer, "weight_coef", amount=0.5)
+    got = _what_linear_gets(monkeypatch, layer)
+    assert torch.equal(got["coefs"], layer.weight_coef_orig * layer.weight_coef_mask) and (got["coefs"] == 0).any()
+
+
+def test_a_coefficient_that_is_a_plain_attribute_is_used(monkeypatch):
+    """As in the replicas of nn.DataParallel, whose parameters are attributes."""
+    layer = SillyLinear(IN, OUT, [K, K], [1, 2], matrix_coef=True)
+    coef = layer.weight_coef.detach().clone()
+    del layer._parameters["weight_coef"]
+    layer.weight_coef = coef
+    assert _what_linear_gets(monkeypatch, layer)["coefs"] is coef
+
+
+@pytest.mark.parametrize("as_parameter", [True, False])
+def test_a_replaced_bias_is_used(as_parameter, monkeypatch):
+    layer = SillyLinear(IN, OUT, [K, K], [1, 2], matrix_coef=True)
+    dense = torch.nn.Parameter(torch.ones(OUT)) if as_parameter else torch.ones(OUT)
+    del layer.bias
+    layer.bias = dense
+    assert _what_linear_gets(monkeypatch, layer)["bias"] is dense
+    layer.bias = None
+    assert _what_linear_gets(monkeypatch, layer)["bias"] is None
+    assert _what_linear_gets(monkeypatch, SillyLinear(IN, OUT, [K, K], [1, 2], matrix_coef=True, bias=False))["bias"] is None

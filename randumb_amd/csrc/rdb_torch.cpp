@@ -8,6 +8,7 @@
 // and workspaces with torch's allocator and calls the library.  Under torch.compile ops.linear takes the registered operators.
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -62,6 +63,19 @@ void same_device(const char *who, const Tensor &at, std::initializer_list<const 
         if (t && t->defined()) check_one(*t);
 }
 const Tensor *address(const OptTensor &t) { return t ? &*t : nullptr; }
+
+// Whether a call on these tensors may go past the dispatcher: not under a mode that wants to see it (tracing, fake tensors, counters),
+// and not on tensors that stand for something else than their memory (fake, batched, tracked by functorch) or carry a forward-mode
+// tangent.  The entry points return None for the others, and their callers take the general path.
+bool past_dispatcher(std::initializer_list<const Tensor *> tensors)
+{
+    static const c10::DispatchKeySet special({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::BatchedNestedTensor,
+                                              c10::DispatchKey::Batched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize});
+    if (c10::impl::TorchDispatchModeTLS::any_modes_set()) return false;
+    for (const Tensor *t : tensors)
+        if (t && t->defined() && (t->key_set().has_any(special) || t->layout() != at::kStrided || t->_fw_grad(0).defined())) return false;
+    return true;
+}
 // What a backward pass gets back of a tensor that it saved.  Saved-tensor hooks put in between may return anything: it is used only
 // if it lies on the gradient's device and is what was saved, as far as the kernels rely on it.
 const Tensor &restored(const char *who, const Tensor &t, const Tensor &grad, at::IntArrayRef sizes)
@@ -831,6 +845,7 @@ void check_sizes(const char *who, const Tensor &x, const Tensor &c, const Layer 
 }
 
 // ----------------------------------------------------------------------------------------------- Python methods
+// They return None for requests that are not to go past the dispatcher (past_dispatcher).
 struct BadArgument {};
 
 const Tensor &tensor_arg(PyObject *o)
@@ -922,6 +937,7 @@ PyObject *py_linear_projected(PyObject *, PyObject *const *a, Py_ssize_t n)
         const OptTensor sb = opt_arg(a[8]);
         same_device("linear_fwd", x, {&c, address(b.coef), address(b.scale), address(sb)});
         check_sizes("linear_fwd", x, c, l, sb, b);
+        if (!past_dispatcher({&x, &c, address(b.coef), address(b.scale), address(sb)})) Py_RETURN_NONE;
         // without a backward pass to come there is no state to keep: the one-call forward
         if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
             return THPVariable_Wrap(linear_fwd(x, c, l, sb, b));
@@ -940,6 +956,7 @@ PyObject *py_linear_one_call(PyObject *, PyObject *const *a, Py_ssize_t n)
         const Bias b = bias_arg(a + 8);
         same_device("linear_fwd", x, {&c, address(b.coef), address(b.scale), address(sb)});
         check_sizes("linear_fwd", x, c, l, sb, b);
+        if (!past_dispatcher({&x, &c, address(b.coef), address(b.scale), address(sb)})) Py_RETURN_NONE;
         if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
             return THPVariable_Wrap(linear_fwd(x, c, l, sb, b));
         return THPVariable_Wrap(OneCallLinear::apply(x, c, sb, b.coef, b.scale, b.seed, l));
@@ -957,6 +974,7 @@ PyObject *py_linear_vector(PyObject *, PyObject *const *a, Py_ssize_t n)
         const Bias b = bias_arg(a + 6);
         same_device("linear_vector", x, {&c, address(b.coef), address(b.scale), address(sb)});
         check_sizes("linear_vector", x, c, l, sb, b);
+        if (!past_dispatcher({&x, &c, address(b.coef), address(b.scale), address(sb)})) Py_RETURN_NONE;
         if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
             return THPVariable_Wrap(VectorLinear::forward(nullptr, x, c, sb, b.coef, b.scale, b.seed, l));
         return THPVariable_Wrap(VectorLinear::apply(x, c, sb, b.coef, b.scale, b.seed, l));
@@ -971,6 +989,8 @@ PyObject *py_embed_rows(PyObject *, PyObject *const *a, Py_ssize_t n)
         const Tensor &idx = tensor_arg(a[0]), &c = tensor_arg(a[1]);
         const int64_t rowsize = int_arg(a[2]), seed = seed_arg(a[3]);
         same_device("embed_fwd", idx, {&c});
+        if (c._fw_grad(0).defined()) fail(PyExc_NotImplementedError, "embed_fwd has no forward-mode derivative");   // the operator would drop it
+        if (!past_dispatcher({&idx, &c})) Py_RETURN_NONE;
         if (!at::GradMode::is_enabled() || !c.requires_grad()) return THPVariable_Wrap(EmbedRows::forward(nullptr, idx, c, rowsize, seed));
         return THPVariable_Wrap(EmbedRows::apply(idx, c, rowsize, seed));
     });
@@ -989,6 +1009,7 @@ PyObject *py_rms_norm(PyObject *, PyObject *const *a, Py_ssize_t n)
     return guarded([&]() -> PyObject * {
         count_args(n, 2);
         const Tensor &x = tensor_arg(a[0]);
+        if (!past_dispatcher({&x})) Py_RETURN_NONE;
         need_bf16("rms_norm", x);
         return THPVariable_Wrap(RmsNorm::apply(x, float_arg(a[1])));
     });
@@ -1000,6 +1021,7 @@ PyObject *py_add_rms_norm(PyObject *, PyObject *const *a, Py_ssize_t n)
     return guarded([&]() -> PyObject * {
         count_args(n, 3);
         const Tensor &x = tensor_arg(a[0]), &delta = tensor_arg(a[1]);
+        if (!past_dispatcher({&x, &delta})) Py_RETURN_NONE;
         need_bf16("add_rms_norm", x);
         need_bf16("add_rms_norm", delta);
         same_device("add_rms_norm", x, {&delta});
@@ -1015,6 +1037,7 @@ PyObject *py_relu_square(PyObject *, PyObject *const *a, Py_ssize_t n)
     return guarded([&]() -> PyObject * {
         count_args(n, 1);
         const Tensor &x = tensor_arg(a[0]);
+        if (!past_dispatcher({&x})) Py_RETURN_NONE;
         need_bf16("relu_square", x);
         return THPVariable_Wrap(ReluSquare::apply(x));
     });
@@ -1026,6 +1049,7 @@ PyObject *py_cross_entropy(PyObject *, PyObject *const *a, Py_ssize_t n)
     return guarded([&]() -> PyObject * {
         count_args(n, 3);
         const Tensor &x = tensor_arg(a[0]), &t = tensor_arg(a[1]);
+        if (!past_dispatcher({&x, &t})) Py_RETURN_NONE;
         need_bf16("cross_entropy", x);
         if (x.dim() != 2 || t.dim() != 1 || t.size(0) != x.size(0) || t.scalar_type() != at::kLong || t.device() != x.device())
             fail(PyExc_ValueError, "cross_entropy needs logits (rows, classes) and int64 targets (rows) on one device");
@@ -1040,6 +1064,7 @@ PyObject *py_causal_attention(PyObject *, PyObject *const *a, Py_ssize_t n)
         count_args(n, 4);
         const Tensor &qkv = tensor_arg(a[0]), &f = tensor_arg(a[1]);
         const int64_t heads = int_arg(a[2]);
+        if (!past_dispatcher({&qkv, &f})) Py_RETURN_NONE;
         need_bf16("causal_attention", qkv);
         if (qkv.dim() != 3 || qkv.size(2) != 3 * heads * 64 || f.numel() != 32 || f.device() != qkv.device())
             fail(PyExc_ValueError, "causal_attention needs qkv (B, T, 3 * heads * 64) and 32 frequencies on one device");

@@ -23,7 +23,8 @@ from .SillyLayers import SillyEmbedding, SillyLinear
 
 
 def _fused(x: torch.Tensor):
-    """The extension module where ``x`` is what its kernels take, else None: bf16 on the GPU, run eagerly."""
+    """The extension module where ``x`` is what its kernels take, else None: bf16 on the GPU, run eagerly.  Its methods return None
+    for tensors that stand for something else than their memory (under a transform or a dispatch mode)."""
     if x.dtype is torch.bfloat16 and x.is_cuda and type(x) in _PLAIN and not torch.compiler.is_compiling() and not torch.is_autocast_enabled():
         return _lib._ext or _lib.extension()
     return None
@@ -39,16 +40,17 @@ def _norm_kernel_takes(x: torch.Tensor) -> bool:
 
 def RT_norm(x: torch.Tensor) -> torch.Tensor:
     ext = _fused(x)
-    if ext is not None and _norm_kernel_takes(x):
-        return ext.rms_norm(x, _EPS)
-    return F.rms_norm(x, (x.size(-1),))
+    y = ext.rms_norm(x, _EPS) if ext is not None and _norm_kernel_takes(x) else None
+    return F.rms_norm(x, (x.size(-1),)) if y is None else y
 
 
 def _add_norm(x: torch.Tensor, delta: torch.Tensor):
     """``x + delta`` and its normalisation."""
     ext = _fused(x)
     if ext is not None and delta.dtype is torch.bfloat16 and delta.shape == x.shape and _norm_kernel_takes(x):
-        return ext.add_rms_norm(x, delta, _EPS)
+        both = ext.add_rms_norm(x, delta, _EPS)
+        if both is not None:
+            return both
     x = x + delta
     return x, RT_norm(x)
 
@@ -107,7 +109,9 @@ class RT_CausalSelfAttention(nn.Module):
         qkv = self.c_qkv(x)
         ext = _fused(qkv)
         if ext is not None and D == 64 * self.n_head and 0 < T * 3 * D < 1 << 29 and B > 0:
-            return self.c_proj(ext.causal_attention(qkv, self.rotary.inv_freq, self.n_head, _EPS))
+            y = ext.causal_attention(qkv, self.rotary.inv_freq, self.n_head, _EPS)
+            if y is not None:
+                return self.c_proj(y)
         q, k, v = qkv.view(B, T, 3, self.n_head, D // self.n_head).unbind(2)
         q, k = RT_norm(q), RT_norm(k)
         q, k = self.rotary(q), self.rotary(k)
@@ -124,7 +128,8 @@ class RT_MLP(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         h = self.c_fc(x)
         ext = _fused(h)
-        return self.c_proj(F.relu(h).square() if ext is None else ext.relu_square(h))
+        a = None if ext is None else ext.relu_square(h)
+        return self.c_proj(F.relu(h).square() if a is None else a)
 
 
 class RT_Block(nn.Module):
@@ -176,6 +181,8 @@ class RT_GPT(nn.Module):
         logits = self.lm_head(RT_norm(x) if normed is None else normed)
         ext = _fused(logits)
         if ext is not None and logits.size(-1) % 8 == 0 and logits.numel() and target.dtype is torch.int64:
-            return ext.cross_entropy(logits.view(-1, logits.size(-1)), target.view(-1), -100)
+            loss = ext.cross_entropy(logits.view(-1, logits.size(-1)), target.view(-1), -100)
+            if loss is not None:
+                return loss
         logits = logits.float()
         return F.cross_entropy(logits.view(-1, logits.size(-1)), target.view(-1))

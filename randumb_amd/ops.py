@@ -263,8 +263,17 @@ def _(dy, state, coefs, in_features, seed):
     return [dy.new_empty([dy.shape[0], in_features]), dy.new_empty([coefs.shape[0], coefs.shape[1]], dtype=torch.float32)]
 
 
+_PLAIN = (Tensor, torch.nn.Parameter)
+
+
 def _tracing() -> bool:
-    return torch.compiler.is_compiling()
+    """Whether calls have to go through the operators: under torch.compile, and under a dispatch mode (fake tensors, tracing)."""
+    return torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
+
+
+def _stands_for_memory(*tensors) -> bool:
+    """False for tensors whose operators are somebody else's (fake tensors, pseudorandom ones, other wrapper subclasses)."""
+    return not any(t is not None and torch._C._dispatch_keys(t).has(torch._C.DispatchKey.Python) for t in tensors)
 
 
 def _dense(t: Optional[Tensor]) -> Optional[Tensor]:
@@ -275,7 +284,8 @@ def _dense(t: Optional[Tensor]) -> Optional[Tensor]:
 
 class _OneCallFunction(torch.autograd.Function):
     """``rten::linear_fwd`` and its registered backward in Python, without the operator wrappers: for the few requests the
-    extension module does not take (a bias that is a pseudorandom tensor of another form than a layer's)."""
+    extension module does not take: a bias that is a pseudorandom tensor of another form than a layer's, and tensors under a
+    transform (forward mode, vmap), which ``autograd.Function`` refuses."""
 
     @staticmethod
     def forward(ctx, x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias):
@@ -376,7 +386,7 @@ class _ProjectedFunction(torch.autograd.Function):
 def _coef_form(t) -> Optional[tuple]:
     """``(coefs, scale or None, seed)`` of a contiguous vector-coef tensor in its coefficients' dtype, as the extension module takes
     a pseudorandom bias or weight (autograd then reaches the coefficients there); None for other pseudorandom tensors."""
-    if t.coef_rows or t.dtype != t._coef.dtype or type(t._coef) not in (Tensor, torch.nn.Parameter) or not t.is_contiguous():
+    if t.coef_rows or t.dtype != t._coef.dtype or type(t._coef) not in _PLAIN or not t.is_contiguous():
         return None
     c, sb = t._coef, t.scale_bias if t.fused_bias else None
     if t.fused_bias and sb is None:
@@ -401,9 +411,8 @@ class _ProjectedLinear:
     @staticmethod
     def apply(x, coefs, in_features, out_features, seed, bias, scale_bias=None):
         form = None if _tracing() or hip.CHECK_STATE_COEF else _bias_form(bias, out_features)
-        if form is None:
-            return _ProjectedFunction.apply(x, coefs, in_features, out_features, seed, bias, scale_bias)
-        return _lib.extension().linear_projected(x, coefs, in_features, out_features, seed, *form, scale_bias)
+        y = None if form is None else _lib.extension().linear_projected(x, coefs, in_features, out_features, seed, *form, scale_bias)
+        return _ProjectedFunction.apply(x, coefs, in_features, out_features, seed, bias, scale_bias) if y is None else y
 
 
 def linear(x: Tensor, coefs: Tensor, in_features: int, out_features: int, stride_o: int, stride_i: int, seed: int,
@@ -411,17 +420,17 @@ def linear(x: Tensor, coefs: Tensor, in_features: int, out_features: int, stride
     """``x @ W.T (+ bias)`` with autograd, choosing the projected form when the layer qualifies (matrix-coef; bf16 with sizes in
     multiples of 8, or fp32 beyond the few-token regime; the fused random bias in bf16 when run eagerly) and
     ``rten::linear_fwd`` otherwise.  Same arguments as ``rten::linear_fwd``."""
-    if x.is_cuda and not _tracing():
+    if not _tracing():
+        if not x.is_cuda or not (type(x) in _PLAIN or _stands_for_memory(x)):
+            return linear_fwd(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias)
         ext = _lib._ext or _lib.extension()
         if ext.takes_projected(x, coefs, in_features, out_features, stride_o, stride_i, scale_bias, bias):
             return _ProjectedLinear.apply(x, coefs, in_features, out_features, seed, bias, scale_bias)
         form = _bias_form(bias, out_features)
-        if form is None:
-            return _OneCallFunction.apply(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias)
-        return ext.linear_one_call(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, *form)
-    rbias_ok = scale_bias is None or (x.dtype == torch.bfloat16 and scale_bias.numel() == 1 and not _tracing()
-                                      and hip.linear_rbias_supported(in_features, out_features, x.dtype))
-    if (rbias_ok and coefs.dim() == 2 and coefs.shape[0] == out_features and stride_o == in_features and stride_i == 1
+        y = None if form is None else ext.linear_one_call(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, *form)
+        return _OneCallFunction.apply(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias) if y is None else y
+    # by operators, which a tracer can follow; the random-bias share has none of its own beside the projected form
+    if (scale_bias is None and coefs.dim() == 2 and coefs.shape[0] == out_features and stride_o == in_features and stride_i == 1
             and x.is_cuda and x.dim() == 2 and x.dtype in (torch.bfloat16, torch.float32) and coefs.dtype == x.dtype
             and (bias is None or bias.dtype == x.dtype)
             and hip.linear_projection_preferred(x.shape[0], in_features, out_features, coefs.shape[1], x.dtype)):
@@ -433,7 +442,7 @@ def vector_linear(x: Tensor, weight, bias) -> Optional[Tensor]:
     """``F.linear(x, weight, bias)`` for a vector-coef weight that is formed and multiplied as a dense matrix, without the tensor
     subclass's dispatch (three operators of torch.library and as many autograd nodes: 480 us of host time for a step whose
     kernels take 60); None where the request is another one."""
-    if (not x.is_cuda or x.dim() < 2 or type(x) not in (Tensor, torch.nn.Parameter) or x.dtype not in (torch.float32, torch.bfloat16)
+    if (not x.is_cuda or x.dim() < 2 or type(x) not in _PLAIN or x.dtype not in (torch.float32, torch.bfloat16)
             or x.dtype != weight.dtype or weight.dim() != 2 or x.shape[-1] != weight.shape[1] or _tracing() or torch.is_autocast_enabled()):
         return None
     if bias is not None and (bias.dtype != x.dtype or bias.shape != (weight.shape[0],)):
@@ -446,9 +455,10 @@ def vector_linear(x: Tensor, weight, bias) -> Optional[Tensor]:
 
 def embed_rows(idx: Tensor, coefs: Tensor, rowsize: int, seed: int) -> Tensor:
     """``rten::embed_fwd`` with its backward; eagerly on the GPU by the extension module."""
+    y = None
     if idx.is_cuda and coefs.is_cuda and not _tracing():
-        return (_lib._ext or _lib.extension()).embed_rows(idx, coefs, rowsize, seed)
-    return embed_fwd(idx, coefs, rowsize, seed)
+        y = (_lib._ext or _lib.extension()).embed_rows(idx, coefs, rowsize, seed)
+    return embed_fwd(idx, coefs, rowsize, seed) if y is None else y
 
 
 # ------------------------------------------------------------------------------------------------ rten_cpp::*

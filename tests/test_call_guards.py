@@ -1,5 +1,7 @@
 """Calls that must be refused before anything is launched, on the CPU: the tensors on "the GPU" are fake ones, which have a device
 and sizes and no memory."""
+import contextlib
+
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
@@ -46,12 +48,6 @@ def test_embedding_with_coefficients_elsewhere_is_refused():
         _lib.extension().embed_rows(_fake(3, dtype=torch.int64), torch.zeros(K), 8, 1)
     with pytest.raises(RuntimeError, match="cuda:1"):
         _lib.extension().embed_rows(_fake(3, dtype=torch.int64), _fake(K, device="cuda:1"), 8, 1)
-
-
-def test_a_layer_that_was_not_moved_is_refused():
-    layer = SillyLinear(IN, OUT, [K, K], [1, 2], matrix_coef=True)
-    with pytest.raises(NotImplementedError, match="CPU implementation"):
-        ops.linear(_fake(4, IN), layer.weight_coef, IN, OUT, IN, 1, 1, None, None)
 
 
 @pytest.mark.parametrize("name", ["scale_bias", "bias"])
@@ -179,3 +175,43 @@ def test_a_replaced_bias_is_used(as_parameter, monkeypatch):
     layer.bias = None
     assert _what_linear_gets(monkeypatch, layer)["bias"] is None
     assert _what_linear_gets(monkeypatch, SillyLinear(IN, OUT, [K, K], [1, 2], matrix_coef=True, bias=False))["bias"] is None
+
+
+# ------------------------------------------------------------------------------------------------ modes, transforms, tangents
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("sizes", [(4, 256, 192, 16), (300, 256, 192, 64), (130, 133, 99, 50)])
+@pytest.mark.parametrize("inside", [True, False])
+def test_fake_tensors_take_the_operators(inside, sizes, dtype):
+    """A layer's output with no GPU and no memory: in the mode and out of it."""
+    tokens, in_f, out_f, k = sizes
+    mode = FakeTensorMode()
+    with mode:
+        x = torch.empty(tokens, in_f, dtype=dtype, device="cuda", requires_grad=True)
+        c = torch.empty(out_f, k, dtype=dtype, device="cuda", requires_grad=True)
+        b = torch.empty(out_f, dtype=dtype, device="cuda")
+    with mode if inside else contextlib.nullcontext():
+        y = ops.linear(x, c, in_f, out_f, in_f, 1, 3, None, b)
+    assert y.shape == (tokens, out_f) and y.dtype == dtype and y.device.type == "cuda"
+
+
+@pytest.mark.parametrize("inside", [True, False])
+def test_fake_indices_take_the_embedding_operator(inside):
+    mode = FakeTensorMode()
+    with mode:
+        idx, c = torch.zeros(3, 5, dtype=torch.int64, device="cuda"), torch.empty(K, device="cuda", requires_grad=True)
+    with mode if inside else contextlib.nullcontext():
+        y = ops.embed_rows(idx, c, 24, 1)
+    assert y.shape == (3, 5, 24)
+
+
+def test_calls_that_do_not_go_past_the_dispatcher():
+    """The extension module's methods leave tensors that stand for something else to their callers."""
+    ext = _lib.extension()
+    x, c, h = _fake(4, IN), _fake(OUT, K), _fake(4, 64, dtype=torch.bfloat16)
+    assert ext.linear_one_call(x, c, IN, OUT, IN, 1, 3, None, None, None, -1) is None
+    assert ext.linear_projected(x, c, IN, OUT, 3, None, None, -1, None) is None
+    assert ext.linear_vector(x, _fake(K), IN, OUT, 3, None, None, None, -1) is None
+    assert ext.embed_rows(_fake(3, dtype=torch.int64), _fake(K), 24, 1) is None
+    assert ext.rms_norm(h, 1e-6) is None and ext.relu_square(h) is None and ext.add_rms_norm(h, h, 1e-6) is None
+    assert ext.cross_entropy(h, _fake(4, dtype=torch.int64), -100) is None
+    assert ext.causal_attention(_fake(1, 4, 192, dtype=torch.bfloat16), _fake(32), 1, 1e-6) is None

@@ -79,3 +79,89 @@ def test_a_layer_and_an_input_on_different_devices_are_refused():
         layer(torch.randn(4, 768, device="cuda"))
     layer = layer.to("cuda")
     assert layer(torch.randn(4, 768, device="cuda")).shape == (4, 96)
+
+
+# ------------------------------------------------------------------------------------------------ modes, transforms, tangents
+@pytest.mark.parametrize("form", [f for f in FORMS if not f.startswith("vector")])
+def test_fake_inputs_of_a_layer_give_fake_outputs(form):
+    from torch._subclasses.fake_tensor import FakeTensor, FakeTensorMode
+
+    layer, x = _layer(form)
+    mode = FakeTensorMode(allow_non_fake_inputs=True)
+    with mode:
+        y = layer(mode.from_tensor(x))
+    assert isinstance(y, FakeTensor) and y.shape == (x.shape[0], layer.out_features) and y.dtype == x.dtype
+
+
+@pytest.mark.parametrize("which", ["x", "coef"])
+@pytest.mark.parametrize("form", [f for f in FORMS if not f.startswith("vector")])
+@torch.no_grad()
+def test_forward_mode_is_refused_not_dropped(form, which):
+    import torch.autograd.forward_ad as fwd
+
+    layer, x = _layer(form)
+    x = x.detach()
+    with fwd.dual_level():
+        if which == "x":
+            x = fwd.make_dual(x, torch.ones_like(x))
+        else:
+            coef = layer.weight_coef.detach()
+            del layer._parameters["weight_coef"]
+            layer.weight_coef = fwd.make_dual(coef, torch.ones_like(coef))
+        with pytest.raises(NotImplementedError, match="jvp"):
+            layer(x)
+
+
+def test_forward_mode_of_the_embedding_is_refused_not_dropped():
+    import torch.autograd.forward_ad as fwd
+
+    e = SillyEmbedding(50, 24, listgen([16]), listgen([3]), device="cuda").requires_grad_(False)
+    with fwd.dual_level():
+        c = e.weight_coef.detach()
+        del e._parameters["weight_coef"]
+        e.weight_coef = fwd.make_dual(c, torch.ones_like(c))
+        with pytest.raises(NotImplementedError, match="forward-mode"):
+            e(torch.tensor([1, 2], device="cuda"))
+
+
+def test_vmap_over_a_layer_is_refused_and_over_the_embedding_runs():
+    layer, x = _layer("one_call_fp32")
+    with pytest.raises(RuntimeError, match="functorch|vmap"):
+        torch.vmap(layer)(x.detach().unsqueeze(1))
+    e = SillyEmbedding(50, 24, listgen([16]), listgen([3]), device="cuda").requires_grad_(False)
+    idx = torch.tensor([[1, 5], [49, 0]], device="cuda")
+    assert torch.equal(torch.vmap(e)(idx), e(idx))
+
+
+def test_forward_mode_through_the_stock_operators_of_a_block():
+    """Normalisation, squared ReLU and the residual sum have forward-mode derivatives in their stock form, which tangents take."""
+    import torch.nn.functional as F
+
+    from randumb_amd import gpt
+
+    x, v = (torch.randn(6, 64, device="cuda").bfloat16() for _ in range(2))
+    for f, stock in ((gpt.RT_norm, lambda t: F.rms_norm(t, (64,))), (lambda t: gpt._add_norm(t, v)[1], lambda t: F.rms_norm(t + v, (64,)))):
+        got, want = torch.func.jvp(f, (x,), (v,)), torch.func.jvp(stock, (x,), (v,))
+        assert torch.equal(got[1], want[1])
+
+
+def test_a_counting_mode_sees_a_layers_products():
+    """A dispatch mode over real tensors sees the operators; the values are those of the direct calls."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Names(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.seen = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    for form, op in (("one_call_fp32", "rten.linear_fwd"), ("projected_bf16", "rten.linear_project_fwd"), ("vector_fp32", "aten.addmm")):
+        layer, x = _layer(form)
+        want = layer(x)
+        with Names() as mode:
+            got = layer(x)
+        assert any(op in n for n in mode.seen), mode.seen
+        assert torch.allclose(got.float(), want.float(), rtol=1e-5, atol=1e-5 * float(want.float().abs().max()))

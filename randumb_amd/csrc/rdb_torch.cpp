@@ -7,11 +7,14 @@
 // 130 us of wall time) and twice what a single-token forward takes.  Nothing here computes: it sizes and allocates outputs
 // and workspaces with torch's allocator and calls the library.  Under torch.compile ops.linear takes the registered operators.
 #include <ATen/ATen.h>
+#include <ATen/core/Reduction.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/autograd.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -622,6 +625,30 @@ class VectorLinear : public Function<VectorLinear> {
     }
 };
 
+// First derivatives computed under create_graph by a function that has no second ones: the first ones are there, going through them
+// again raises (a result without a graph would pass for one that does not depend on the inputs).  varies: whether something the
+// derivative depends on has a gradient to come.
+Tensor once_differentiable(const char *who, const Tensor &grad, bool varies)
+{
+    if (!at::GradMode::is_enabled() || !varies) return grad;
+    auto error = std::make_shared<torch::autograd::DelayedError>(std::string(who) + " has no second derivative", 1);
+    return (*error)({grad.detach().set_requires_grad(true)})[0];
+}
+// Gradient of f(inputs...) with a graph of its own (create_graph), by f's stock operators.  Inputs without a gradient to come: undefined
+template <typename F> variable_list stock_gradient(F f, const variable_list &inputs, const variable_list &grads)
+{
+    variable_list wanted;
+    for (const Tensor &t : inputs)
+        if (t.requires_grad()) wanted.push_back(t);
+    variable_list out(inputs.size());
+    if (wanted.empty()) return out;
+    const variable_list got = torch::autograd::grad(f(inputs), wanted, grads, true, true, true);
+    size_t n = 0;
+    for (size_t i = 0; i < inputs.size(); ++i)
+        if (inputs[i].requires_grad()) out[i] = got[n++];
+    return out;
+}
+
 // rows idx of a (*, rowsize) vector-coef table, fp32
 class EmbedRows : public Function<EmbedRows> {
   public:
@@ -650,8 +677,12 @@ class EmbedRows : public Function<EmbedRows> {
     {
         const Tensor idx = ctx->get_saved_variables()[0];
         const auto m = ctx->saved_data["m"].toIntVector();
+        return {Tensor(), once_differentiable("embed_fwd", gradient(idx, grads[0], m), grads[0].requires_grad()), Tensor(), Tensor()};
+    }
+    static Tensor gradient(const Tensor &idx, const Tensor &grad, const std::vector<int64_t> &m)
+    {
         const at::AutoGradMode no_grad(false);
-        const Tensor d = native(grads[0]);
+        const Tensor d = native(grad);
         restored_values("embedding (backward)", idx, d, at::kLong, m[1] ? d.numel() / m[1] : 0);
         const c10::OptionalDeviceGuard guard(d.device());
         Tensor dc = at::empty({m[0]}, d.options().dtype(at::kFloat));
@@ -660,7 +691,7 @@ class EmbedRows : public Function<EmbedRows> {
         check(rdb_embed_bwd(dc.data_ptr<float>(), idx.data_ptr<int64_t>(), idx.numel(), d.data_ptr(), code(d.scalar_type()), m[0], m[1], (uint32_t)m[2], ptr(ws),
                             need, stream_of(d)),
               "rdb_embed_bwd");
-        return {Tensor(), dc.to((at::ScalarType)m[3]), Tensor(), Tensor()};
+        return dc.to((at::ScalarType)m[3]);
     }
 };
 
@@ -672,6 +703,8 @@ void need_bf16(const char *who, const Tensor &t)
 }
 int64_t row_count(const Tensor &x) { return x.size(-1) ? x.numel() / x.size(-1) : 0; }
 
+// A gradient asked for under create_graph is computed by the stock operators, from the inputs as they were given.
+
 // x -> x / rms(x) over the last dimension
 class RmsNorm : public Function<RmsNorm> {
   public:
@@ -682,16 +715,23 @@ class RmsNorm : public Function<RmsNorm> {
         Tensor y = at::empty_like(x), rstd = at::empty({row_count(x)}, x.options().dtype(at::kFloat));
         check(rdb_rms_norm_fwd(y.data_ptr(), nullptr, rstd.data_ptr<float>(), x.data_ptr(), nullptr, row_count(x), x.size(-1), (float)eps, stream_of(x)),
               "rdb_rms_norm_fwd");
-        ctx->save_for_backward({x, rstd});
+        ctx->save_for_backward({x0, rstd});
+        ctx->saved_data["eps"] = eps;
         return y;
     }
+    static Tensor stock(const Tensor &x, double eps) { return at::rms_norm(x, {x.size(-1)}, {}, eps); }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
         const auto saved = ctx->get_saved_variables();
-        const at::AutoGradMode no_grad(false);
-        const Tensor &x = saved[0], dy = grads[0].contiguous();
-        restored_values("rms_norm (backward)", x, dy, at::kBFloat16, dy.numel());
-        restored_values("rms_norm (backward)", saved[1], dy, at::kFloat, row_count(dy));
+        constexpr const char *who = "rms_norm (backward)";
+        restored(who, saved[0], grads[0], grads[0].sizes());
+        if (at::GradMode::is_enabled()) {
+            const double eps = ctx->saved_data["eps"].toDouble();
+            return {stock_gradient([&](const variable_list &in) { return variable_list{stock(in[0], eps)}; }, {saved[0]}, {grads[0]})[0], Tensor()};
+        }
+        const Tensor x = saved[0].contiguous(), dy = grads[0].contiguous();
+        restored_values(who, x, dy, at::kBFloat16, dy.numel());
+        restored_values(who, saved[1], dy, at::kFloat, row_count(dy));
         const c10::OptionalDeviceGuard guard(x.device());
         Tensor dx = at::empty_like(x);
         check(rdb_rms_norm_bwd(dx.data_ptr(), dy.data_ptr(), x.data_ptr(), nullptr, saved[1].data_ptr<float>(), row_count(x), x.size(-1), stream_of(x)),
@@ -712,17 +752,26 @@ class AddRmsNorm : public Function<AddRmsNorm> {
                                stream_of(x)),
               "rdb_rms_norm_fwd");
         ctx->save_for_backward({sum, rstd});
+        ctx->saved_data["eps"] = eps;
         ctx->set_materialize_grads(false);
         return {sum, y};
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
         const auto saved = ctx->get_saved_variables();
-        const at::AutoGradMode no_grad(false);
         if (!grads[1].defined()) return {grads[0], grads[0], Tensor()};
-        const Tensor &x = saved[0], dy = grads[1].contiguous(), dsum = grads[0].defined() ? grads[0].contiguous() : Tensor();
-        restored_values("add_rms_norm (backward)", x, dy, at::kBFloat16, dy.numel());
-        restored_values("add_rms_norm (backward)", saved[1], dy, at::kFloat, row_count(dy));
+        const Tensor &x = saved[0];   // the sum: an output, with this function behind it
+        constexpr const char *who = "add_rms_norm (backward)";
+        restored(who, x, grads[1], grads[1].sizes());
+        if (at::GradMode::is_enabled()) {
+            const double eps = ctx->saved_data["eps"].toDouble();
+            Tensor d = stock_gradient([&](const variable_list &in) { return variable_list{RmsNorm::stock(in[0], eps)}; }, {x}, {grads[1]})[0];
+            if (d.defined() && grads[0].defined()) d = d + grads[0];
+            return {d, d, Tensor()};
+        }
+        const Tensor dy = grads[1].contiguous(), dsum = grads[0].defined() ? grads[0].contiguous() : Tensor();
+        restored_values(who, x, dy, at::kBFloat16, dy.numel());
+        restored_values(who, saved[1], dy, at::kFloat, row_count(dy));
         const c10::OptionalDeviceGuard guard(x.device());
         Tensor dx = at::empty_like(x);
         check(rdb_rms_norm_bwd(dx.data_ptr(), dy.data_ptr(), x.data_ptr(), ptr(dsum), saved[1].data_ptr<float>(), row_count(x), x.size(-1), stream_of(x)),
@@ -739,15 +788,18 @@ class ReluSquare : public Function<ReluSquare> {
         const c10::OptionalDeviceGuard guard(x.device());
         Tensor y = at::empty_like(x);
         check(rdb_relu_square(y.data_ptr(), x.data_ptr(), nullptr, x.numel(), stream_of(x)), "rdb_relu_square");
-        ctx->save_for_backward({x});
+        ctx->save_for_backward({x0});
         return y;
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
-        const Tensor x = ctx->get_saved_variables()[0];
-        const at::AutoGradMode no_grad(false);
-        const Tensor dy = grads[0].contiguous();
-        restored_values("relu_square (backward)", x, dy, at::kBFloat16, dy.numel());
+        const Tensor x0 = ctx->get_saved_variables()[0];
+        constexpr const char *who = "relu_square (backward)";
+        restored(who, x0, grads[0], grads[0].sizes());
+        if (at::GradMode::is_enabled())
+            return stock_gradient([](const variable_list &in) { return variable_list{at::relu(in[0]).square()}; }, {x0}, {grads[0]});
+        const Tensor x = x0.contiguous(), dy = grads[0].contiguous();
+        restored_values(who, x, dy, at::kBFloat16, dy.numel());
         const c10::OptionalDeviceGuard guard(x.device());
         Tensor dx = at::empty_like(x);
         check(rdb_relu_square(dx.data_ptr(), x.data_ptr(), dy.data_ptr(), x.numel(), stream_of(x)), "rdb_relu_square");
@@ -767,19 +819,25 @@ class CrossEntropy : public Function<CrossEntropy> {
         check(rdb_cross_entropy_fwd(loss.data_ptr<float>(), scratch.data_ptr<float>(), logits.data_ptr(), target.data_ptr<int64_t>(), rows, logits.size(1), ignore,
                                     stream_of(logits)),
               "rdb_cross_entropy_fwd");
-        ctx->save_for_backward({logits, target, scratch});
+        ctx->save_for_backward({logits0, target, scratch});
         ctx->saved_data["m"] = std::vector<int64_t>{rows, logits.size(1), ignore};
         return loss;
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
         const auto saved = ctx->get_saved_variables();
-        const at::AutoGradMode no_grad(false);
-        const Tensor &logits = saved[0], dloss = grads[0].to(at::kFloat).contiguous();
         const auto m = ctx->saved_data["m"].toIntVector();   // rows, classes, ignored label
         constexpr const char *who = "cross_entropy (backward)";
-        restored(who, restored_values(who, logits, dloss, at::kBFloat16, m[0] * m[1]), dloss, {m[0], m[1]});
-        restored_values(who, saved[1], dloss, at::kLong, m[0]);
+        restored(who, saved[0], grads[0], {m[0], m[1]});
+        restored_values(who, saved[1], grads[0], at::kLong, m[0]);
+        if (at::GradMode::is_enabled()) {
+            const auto loss = [&](const variable_list &in) {
+                return variable_list{at::cross_entropy_loss(in[0].to(at::kFloat), saved[1], {}, at::Reduction::Mean, m[2])};
+            };
+            return {stock_gradient(loss, {saved[0]}, {grads[0]})[0], Tensor(), Tensor()};
+        }
+        const Tensor logits = saved[0].contiguous(), dloss = grads[0].to(at::kFloat).contiguous();
+        restored_values(who, logits, dloss, at::kBFloat16, m[0] * m[1]);
         restored_values(who, saved[2], dloss, at::kFloat, 2 * m[0] + 1);
         const c10::OptionalDeviceGuard guard(logits.device());
         Tensor d = at::empty_like(logits);
@@ -811,8 +869,12 @@ class CausalAttention : public Function<CausalAttention> {
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
         const auto saved = ctx->get_saved_variables();
+        return {once_differentiable("causal_attention", gradient(ctx, saved, grads[0]), true), Tensor(), Tensor(), Tensor()};   // qkv is an input of it
+    }
+    static Tensor gradient(AutogradContext *ctx, const variable_list &saved, const Tensor &grad)
+    {
         const at::AutoGradMode no_grad(false);
-        const Tensor &qkv = saved[0], dy = grads[0].contiguous();
+        const Tensor &qkv = saved[0], dy = grad.contiguous();
         constexpr const char *who = "causal_attention (backward)";
         const int64_t B = dy.size(0), T = dy.size(1), heads = ctx->saved_data["heads"].toInt();
         restored(who, restored_values(who, qkv, dy, at::kBFloat16, 3 * dy.numel()), dy, {B, T, 3 * heads * 64});
@@ -824,7 +886,7 @@ class CausalAttention : public Function<CausalAttention> {
                                        qkv.data_ptr(), B, T, heads, (float)ctx->saved_data["eps"].toDouble(),
                                        stream_of(qkv)),
               "rdb_causal_attention_bwd");
-        return {d, Tensor(), Tensor(), Tensor()};
+        return d;
     }
 };
 

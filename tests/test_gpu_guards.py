@@ -165,3 +165,48 @@ def test_a_counting_mode_sees_a_layers_products():
             got = layer(x)
         assert any(op in n for n in mode.seen), mode.seen
         assert torch.allclose(got.float(), want.float(), rtol=1e-5, atol=1e-5 * float(want.float().abs().max()))
+
+
+# ------------------------------------------------------------------------------------------------ second derivatives
+@pytest.mark.parametrize("strided", [False, True])
+@pytest.mark.parametrize("op", ["rms_norm", "add_rms_norm", "relu_square", "cross_entropy"])
+def test_second_derivatives_of_a_blocks_operators(op, strided):
+    """First derivatives under create_graph, and the derivatives of those, are the stock operators' in bf16 (the same kernels)."""
+    import torch.nn.functional as F
+
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(64, 40, device="cuda", generator=g).bfloat16()
+    x = (x.t() if strided else x.t().contiguous()).requires_grad_()           # 40 rows of 64
+    d = torch.randn(40, 64, device="cuda", generator=g).bfloat16().requires_grad_()
+    t = torch.randint(0, 64, (40,), device="cuda", generator=g)
+    w = torch.randn(40, 64, device="cuda", generator=g).bfloat16().requires_grad_()   # the incoming gradient, differentiated as well
+    ext, eps = _lib.extension(), torch.finfo(torch.float32).eps
+    fused, stock, inputs = {
+        "rms_norm": (lambda: ext.rms_norm(x, eps), lambda: F.rms_norm(x, (64,)), [x, w]),
+        "add_rms_norm": (lambda: sum(ext.add_rms_norm(x, d, eps)), lambda: (x + d) + F.rms_norm(x + d, (64,)), [x, d, w]),
+        "relu_square": (lambda: ext.relu_square(x), lambda: F.relu(x).square(), [x, w]),
+        "cross_entropy": (lambda: ext.cross_entropy(x, t, -100), lambda: F.cross_entropy(x.float(), t), [x]),
+    }[op]
+
+    def both(f):
+        y = f()
+        first = torch.autograd.grad(y, [i for i in inputs if i is not w], w if y.dim() else None, create_graph=True)
+        return [*first, *torch.autograd.grad(sum((p.float() ** 2).sum() for p in first), inputs)]
+
+    for a, b in zip(both(fused), both(stock)):
+        assert a.shape == b.shape and torch.linalg.vector_norm((a - b).double()) <= 1e-2 * torch.linalg.vector_norm(b.double())
+
+
+def test_second_derivatives_that_do_not_exist_raise():
+    e = SillyEmbedding(50, 24, listgen([16]), listgen([3]), device="cuda")
+    w = torch.randn(2, 24, device="cuda", requires_grad=True)
+    y = e(torch.tensor([1, 5], device="cuda"))
+    (first,) = torch.autograd.grad(y, e.weight_coef, w, create_graph=True)
+    assert torch.equal(first.detach(), torch.autograd.grad(e(torch.tensor([1, 5], device="cuda")), e.weight_coef, w.detach())[0])
+    with pytest.raises(RuntimeError, match="second derivative"):
+        first.sum().backward()
+    qkv = torch.randn(1, 8, 192, device="cuda").bfloat16().requires_grad_()
+    y = _lib.extension().causal_attention(qkv, torch.ones(32, device="cuda"), 1, 1e-6)
+    (first,) = torch.autograd.grad(y, qkv, torch.ones_like(y), create_graph=True)
+    with pytest.raises(RuntimeError, match="second derivative"):
+        first.float().sum().backward()

@@ -149,9 +149,13 @@ class RT_Block(nn.Module):
         return _add_norm(x, self.mlp(h))
 
     def _plain(self) -> bool:
-        """Nothing that has to see ``forward`` run: no subclass, no replaced method, no hooks."""
-        return (type(self) is RT_Block and "forward" not in self.__dict__ and not torch.nn.modules.module._has_any_global_hook()
+        """Nothing that has to see ``forward`` run: no subclass, no replaced method, no compiled call, no hooks."""
+        return (type(self) is RT_Block and "forward" not in self.__dict__ and RT_Block.forward is _BLOCK_FORWARD and RT_Block.__call__ is _MODULE_CALL
+                and self._compiled_call_impl is None and not torch.nn.modules.module._has_any_global_hook()
                 and not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks or self._backward_pre_hooks))
+
+
+_BLOCK_FORWARD, _MODULE_CALL = RT_Block.forward, nn.Module.__call__   # as they stand here: replaced ones are called
 
 
 class RT_GPT(nn.Module):

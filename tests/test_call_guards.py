@@ -215,3 +215,39 @@ def test_calls_that_do_not_go_past_the_dispatcher():
     assert ext.rms_norm(h, 1e-6) is None and ext.relu_square(h) is None and ext.add_rms_norm(h, h, 1e-6) is None
     assert ext.cross_entropy(h, _fake(4, dtype=torch.int64), -100) is None
     assert ext.causal_attention(_fake(1, 4, 192, dtype=torch.bfloat16), _fake(32), 1, 1e-6) is None
+
+
+# ------------------------------------------------------------------------------------------------ blocks whose forward has to run
+def test_blocks_whose_call_somebody_replaced_are_called(monkeypatch):
+    """RT_GPT hands plain blocks each other's normalisation instead of calling them; whatever has to see the call gets it."""
+    from randumb_amd.gpt import RT_Block, RT_GPT, RT_GPTConfig
+
+    model = RT_GPT(RT_GPTConfig(int_dim_gen=iter([8] * 8), seed_gen=iter(range(8)), vocab_size=64, n_layer=2, n_head=2, n_embd=64))
+    block = model.h[0]
+    assert block._plain()
+
+    class Other(RT_Block):
+        pass
+
+    def forward(self, x):
+        return x
+
+    with monkeypatch.context() as m:
+        m.setattr(RT_Block, "forward", forward)
+        assert not block._plain()
+    with monkeypatch.context() as m:
+        m.setattr(RT_Block, "__call__", forward, raising=False)
+        assert not block._plain()
+    block.forward = lambda x: x
+    assert not block._plain()
+    del block.forward
+    with monkeypatch.context() as m:
+        m.setattr(block, "__class__", Other)
+        assert not block._plain()
+    for register in ("register_forward_hook", "register_forward_pre_hook", "register_full_backward_hook", "register_full_backward_pre_hook"):
+        hook = getattr(block, register)(lambda *a: None)
+        assert not block._plain()
+        hook.remove()
+    assert block._plain()
+    block.compile()
+    assert not block._plain() and model.h[1]._plain()

@@ -435,8 +435,8 @@ int rdb_rms_norm_bwd(void *dx, const void *dy, const void *x, const void *dsum, 
 int rdb_relu_square(void *out, const void *x, const void *dy, int64_t n, void *stream);
 
 /* loss[0] (fp32) = mean over the rows with target != ignore_index of log(sum exp(logits[row])) - logits[row][target[row]].
- * scratch: 2 * rows + 1 floats; its first rows + 1 are what the backward call needs.  A target outside the classes gives NaN.
- * classes a multiple of 8, 16-byte aligned logits (RDB_E_UNSUPPORTED otherwise). */
+ * scratch: 2 * rows + 1 floats; its first rows + 1 are what the backward call needs.  A target outside the classes gives NaN,
+ * in the loss and in its row of dlogits.  classes a multiple of 8, 16-byte aligned logits (RDB_E_UNSUPPORTED otherwise). */
 int rdb_cross_entropy_fwd(float *loss, float *scratch, const void *logits, const int64_t *target, int64_t rows, int64_t classes,
                           int64_t ignore_index, void *stream);
 int rdb_cross_entropy_bwd(void *dlogits, const void *logits, const int64_t *target, const float *scratch, const float *dloss,

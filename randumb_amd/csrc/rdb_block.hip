@@ -251,7 +251,8 @@ __global__ __launch_bounds__(1024) void cross_entropy_mean_kernel(float *__restr
     }
 }
 
-// dlogits = (exp(logit - lse) - [class == target]) * dloss / count, 0 in ignored rows
+// dlogits = (exp(logit - lse) - [class == target]) * dloss / count, 0 in ignored rows, NaN in rows whose target is outside the
+// classes (their loss is NaN too: a program that does not look at the loss must not train on them)
 __global__ __launch_bounds__(256) void cross_entropy_bwd_kernel(bf16_t *__restrict__ dlogits, const bf16_t *__restrict__ logits,
                                                                 const int64_t *__restrict__ target, const float *__restrict__ lse,
                                                                 const float *__restrict__ dloss, const float *__restrict__ count, int64_t V, int64_t ignore)
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(256) void cross_entropy_bwd_kernel(bf16_t *__restri
     const int64_t row = blockIdx.x, c = target[row];
     const u32x4 *rv = reinterpret_cast<const u32x4 *>(logits + row * V);
     u32x4 *ov = reinterpret_cast<u32x4 *>(dlogits + row * V);
-    const float l = lse[row] * LOG2E, g = c == ignore ? 0.0f : dloss[0] / count[0];
+    const float l = lse[row] * LOG2E, g = c == ignore ? 0.0f : c < 0 || c >= V ? __uint_as_float(0x7fc00000u) : dloss[0] / count[0];
     const int nvec = (int)(V / 8);
 #pragma unroll 4
     for (int i = threadIdx.x; i < nvec; i += 256) {

@@ -83,6 +83,22 @@ def test_cross_entropy(ext, rows, classes):
     assert bool(ext.cross_entropy(x, torch.full_like(t, classes), -100).isnan())
 
 
+@pytest.mark.parametrize("label", [-1, 2056, 1 << 40, -(1 << 40)])
+def test_a_label_outside_the_classes_does_not_train(ext, label):
+    """Its loss is NaN and so is its row of the gradient; the other rows' gradients are what they are."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = bf16(g, 9, 2056).requires_grad_()
+    t = torch.randint(0, 2056, (9,), generator=g, device="cuda")
+    t[3] = -100
+    (ref,) = torch.autograd.grad(ext.cross_entropy(x, t, -100), x)
+    t[4] = label
+    loss = ext.cross_entropy(x, t, -100)
+    (got,) = torch.autograd.grad(loss, x)
+    assert bool(loss.isnan()) and bool(got[4].isnan().all())
+    rest = [i for i in range(9) if i != 4]
+    assert torch.equal(got[rest], ref[rest]) and not bool(got[3].any())
+
+
 def _attention(qkv, inv_freq, H):
     """The stock operators of RT_CausalSelfAttention, in qkv's precision, with q, k rounded to bf16 as they are there."""
     from randumb_amd.gpt import Rotary

@@ -137,8 +137,9 @@ __device__ __forceinline__ uint32_t relu2_pair(uint32_t w)
 }
 __device__ __forceinline__ uint32_t relu2_grad_pair(uint32_t w, uint32_t d)
 {
+    // 0 where x <= 0 whatever dy is, an infinite or undefined one included
     const float a = relu(lo_f32(w)), b = relu(hi_f32(w));
-    return f32x2_to_bf16x2(lo_f32(d) * (a + a), hi_f32(d) * (b + b));
+    return f32x2_to_bf16x2(a == 0.0f ? 0.0f : lo_f32(d) * (a + a), b == 0.0f ? 0.0f : hi_f32(d) * (b + b));
 }
 
 template <bool GRAD> __global__ __launch_bounds__(256) void relu_square_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ x,

@@ -61,6 +61,15 @@ def test_relu_square_is_the_stock_chain_bit_for_bit(ext, n):
     assert torch.equal(ga.nan_to_num(7), gb.nan_to_num(7))
 
 
+def test_relu_square_with_gradients_that_are_not_finite(ext):
+    """Where x <= 0 the stock operators pass nothing on, an infinite gradient included."""
+    v = torch.tensor([-2.0, -0.0, 0.0, 1.5, math.inf, -math.inf, math.nan], device="cuda").bfloat16()
+    x, dy = (t.flatten() for t in torch.meshgrid(v, v, indexing="ij"))
+    a, b = x.clone().requires_grad_(), x.clone().requires_grad_()
+    ga, gb = torch.autograd.grad(ext.relu_square(a), a, dy)[0], torch.autograd.grad(F.relu(b).square(), b, dy)[0]
+    assert torch.equal(ga.isnan(), gb.isnan()) and torch.equal(ga.nan_to_num(7), gb.nan_to_num(7))
+
+
 @pytest.mark.parametrize("rows,classes", [(1, 8), (3, 64), (130, 2056), (1025, 4096), (64, 50304)])
 def test_cross_entropy(ext, rows, classes):
     print(f"case cross entropy {rows} x {classes}", flush=True)

@@ -132,6 +132,14 @@ Tensor act(const Tensor &t0)
     return t.stride(1) == 1 && t.stride(0) >= t.size(1) ? t : t.contiguous();
 }
 
+// ... whose rows lie no farther apart than one launch addresses (2^29 elements): slices of very wide matrices are copied.  For the
+// calls that keep something for the backward pass; the others fall through to kernels that take any stride.
+Tensor near_act(const Tensor &t0)
+{
+    const Tensor t = act(t0);
+    return t.size(0) * t.stride(0) >= (1ll << 29) ? t.contiguous() : t;
+}
+
 Tensor bytes(int64_t n, const Tensor &like) { return n > 0 ? at::empty({n}, like.options().dtype(at::kByte)) : Tensor(); }
 void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
 
@@ -325,8 +333,9 @@ class OneCallLinear : public Function<OneCallLinear> {
         }
         const c10::OptionalDeviceGuard guard(x.device());
         const Tensor c = coefs.contiguous(), sb = scale_bias ? scale_bias->to(c.scalar_type()) : Tensor(), bv = b.values(l.out_f, x.scalar_type());
+        const Tensor xn = near_act(x);
         Tensor y = at::empty({x.size(0), l.out_f}, x.options()), kept = bytes(keep, x);
-        check(rdb_linear_fwd_kept(y.data_ptr(), l.out_f, kept.data_ptr(), x.data_ptr(), x.stride(0), c.data_ptr(), ptr(sb), ptr(bv), &d, stream_of(x)),
+        check(rdb_linear_fwd_kept(y.data_ptr(), l.out_f, kept.data_ptr(), xn.data_ptr(), xn.stride(0), c.data_ptr(), ptr(sb), ptr(bv), &d, stream_of(x)),
               "rdb_linear_fwd_kept");
         ctx->save_for_backward({scale_bias ? x0 : Tensor(), coefs, scale_bias.value_or(Tensor()), kept});
         return y;
@@ -345,12 +354,12 @@ class OneCallLinear : public Function<OneCallLinear> {
         const at::AutoGradMode no_grad(false);
         const bool want_dx = ctx->needs_input_grad(0), want_dc = ctx->needs_input_grad(1);
         bool want_sb = has_sb && ctx->needs_input_grad(2);
-        const Tensor dy = kept.defined() ? act(grads[0]) : grads[0].contiguous();
+        const Tensor dy = kept.defined() ? near_act(grads[0]) : grads[0].contiguous();
         Tensor dx, dc, dsb;
         if (kept.defined()) {
             if (want_dx || want_dc || want_sb) {
                 const c10::OptionalDeviceGuard guard(dy.device());
-                const Tensor c = coefs.contiguous(), xs = want_sb ? act(x) : Tensor(), s = has_sb ? sb.to(c.scalar_type()) : Tensor();
+                const Tensor c = coefs.contiguous(), xs = want_sb ? near_act(x) : Tensor(), s = has_sb ? sb.to(c.scalar_type()) : Tensor();
                 const rdb_linear_desc d = desc(dy, l, c);
                 const int64_t kept_bytes = rdb_linear_kept_bytes(&d);   // 0: the coefficients came back in another dtype
                 restored_values(who, kept, dy, at::kByte, kept_bytes ? kept_bytes : -1);
@@ -397,7 +406,7 @@ class ProjectedLinear : public Function<ProjectedLinear> {
                           const OptTensor &scale_bias, const Layer &l)
     {
         const Bias pb{bias, bias_scale, bias_seed};
-        const Tensor x = act(x0), c = coefs.contiguous();
+        const Tensor x = near_act(x0), c = coefs.contiguous();
         const c10::OptionalDeviceGuard guard(x.device());
         const rdb_linear_desc d = desc(x, l, c);
         const int64_t need = rdb_linear_projection_bytes(&d);
@@ -442,7 +451,7 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         const at::AutoGradMode no_grad(false);
         const bool want_x = ctx->needs_input_grad(0), want_dc = ctx->needs_input_grad(1), want_sb = has_sb && ctx->needs_input_grad(2 + m[4]);
         const bool want_dx = want_x || want_sb;   // the gradient of the scale comes out of the random-bias share of dx
-        Tensor dy = act(grads[0]);
+        Tensor dy = near_act(grads[0]);
         const bool f32 = coefs.scalar_type() == at::kFloat;
         if (!f32 && (dy.stride(0) % 8 || (uintptr_t)dy.data_ptr() % 16)) dy = dy.contiguous();   // rows with a leading dimension are read in place
         const Tensor c = coefs.contiguous();
@@ -473,7 +482,7 @@ class ProjectedLinear : public Function<ProjectedLinear> {
             dc = dc.to(c.scalar_type());
         }
         if (has_sb && dx.defined()) {
-            const Tensor x = act(saved[3]), sb = native(scale_bias).to(at::kBFloat16);
+            const Tensor x = near_act(saved[3]), sb = native(scale_bias).to(at::kBFloat16);
             const rdb_linear_desc r = rbias_desc(dy, l);
             const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_BWD_FULL, &r);
             const Tensor ws = bytes(need, dy);

@@ -210,3 +210,26 @@ def test_second_derivatives_that_do_not_exist_raise():
     (first,) = torch.autograd.grad(y, qkv, torch.ones_like(y), create_graph=True)
     with pytest.raises(RuntimeError, match="second derivative"):
         first.float().sum().backward()
+
+
+# ------------------------------------------------------------------------------------------------ slices of very wide matrices
+@pytest.mark.parametrize("sliced", ["x", "dy"])
+@pytest.mark.parametrize("form", ["projected_bf16", "projected_fp32", "random_bias_bf16", "kept_bf16"])
+def test_rows_farther_apart_than_one_launch_addresses(form, sliced):
+    """2^29 elements from the first row to the last: the layer runs, with the results of a contiguous input."""
+    layer, x = _layer(form)
+    wanted = [x, *[p for n, p in layer.named_parameters() if "scale" not in n or form.startswith("random")]]
+    dy = torch.randn(x.shape[0], layer.out_features, device="cuda").to(x.dtype)
+    y = layer(x)
+    ref = [y.detach(), *torch.autograd.grad(y, wanted, dy)]
+
+    def spread(t):
+        wide = torch.empty(t.shape[0], (1 << 29) // t.shape[0] // 8 * 8 + 8, device="cuda", dtype=t.dtype)[:, : t.shape[1]]
+        return wide.copy_(t)
+
+    wanted[0] = x2 = spread(x.detach()).requires_grad_() if sliced == "x" else x
+    assert x2.shape[0] * x2.stride(0) >= 1 << 29 or sliced == "dy"
+    y = layer(x2)
+    got = [y.detach(), *torch.autograd.grad(y, wanted, spread(dy) if sliced == "dy" else dy)]
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)

@@ -108,8 +108,8 @@ int64_t rdb_bias_bwd_workspace_bytes(int64_t rows, int64_t n);
  * The dense products around a materialised weight (aten.mm of R.py:942-946 and its backward), fp32:
  *   out[M x N] = A . B^T (+ bias[N]),  A [M x K], B [N x K] row-major; a_across / b_across: stored transposed, [K x M] / [K x N].
  * out is contiguous.  (0, 0), (0, 1) and (1, 1) of the across flags.  On the bf16 matrix cores at fp32 accuracy (three-way
- * split of both sides, see rdb_set_f32_split); an infinite input becomes NaN.  The workspace holds partial sums over ranges of
- * K, added in a fixed order; with less of it (or a bias) fewer ranges run.  RDB_E_UNSUPPORTED: empty, or 2^29 elements or more. */
+ * split of both sides, see rdb_set_f32_split; infinities and NaNs as in an fp32 product).  The workspace holds partial sums over ranges
+ * of K, added in a fixed order; with less of it (or a bias) fewer ranges run.  RDB_E_UNSUPPORTED: empty, or 2^29 elements or more. */
 int rdb_product_f32(float *out, const float *a, int64_t lda, int a_across, const float *b, int64_t ldb, int b_across,
                     const float *bias, int64_t M, int64_t N, int64_t K, void *workspace, int64_t workspace_bytes,
                     void *stream);
@@ -389,7 +389,8 @@ int rdb_set_big_tiles(int mode);
  * product runs as six bf16 matrix instructions (ah bh + ah bm + am bh + ah bl + al bh + am bm, fp32 accumulation): the terms
  * left out are below 2^-23 of a product, an fp32 multiplication's own rounding, and the 32 x 32 x 16 bf16 instruction does in
  * 3/8 of the time what eight 32 x 32 x 2 fp32 ones do.  mode 0: fp32 matrix instructions.  Results agree to fp32 rounding;
- * with mode 1 an infinite input gives NaN where mode 0 gives an infinity.  Process-wide; returns the previous mode. */
+ * infinities and NaNs in fp32 matrices come out as they do in mode 0, an infinity in a bf16 matrix (odd-sized bf16 layers) may
+ * come out as NaN.  Process-wide; returns the previous mode. */
 int rdb_set_f32_split(int mode);
 
 /* ------------------------------------------------------------------------------- one-launch forms and their bounded waits

@@ -53,16 +53,24 @@ struct FgParams {
 };
 
 // fp32 products on the bf16 matrix cores.  v = h + m + l exactly, each part a bf16 (the top 8 bits of what is left: truncation,
-// so every difference is exact); a product a . b is then the sum of the nine products of the parts, each exact in the matrix
-// core's fp32 accumulation, and the six largest of them, ah bh + ah bm + am bh + ah bl + al bh + am bm, leave out less than
-// 2^-23 |a b|: an fp32 product's own rounding.  Six bf16 matrix instructions of 32 x 32 x 16 do the work of eight fp32 ones of
-// 32 x 32 x 2 in 3/8 of the time.  (An infinite input becomes NaN: inf - inf.)  The parts come back as fp32 bit patterns with
-// the low half zero.
-__device__ __forceinline__ void fg_split3(float v, uint32_t &h, uint32_t &m, uint32_t &l)
+// so every difference is exact and the parts have v's sign).  A product a . b is then the sum of the nine products of the parts, each
+// exact in the matrix core's fp32 accumulation, of which the six largest are computed: ah bh + ah bm + am bh + ah bl + al bh + am bm.
+// The three left out, am bl + al bm + al bl, are less than 1.01 * 2^-21 |a b| (|m| < 2^-7 |v|, |l| < 2^-15 |v|; a = b = 1 + 2^-7 - 2^-23
+// comes to 2^-21.03), 2^-24.5 |a b| on average over normally distributed values.  Six bf16 matrix instructions of 32 x 32 x 16 do
+// the work of eight fp32 ones of 32 x 32 x 2 in 3/8 of the time.  The parts come back as fp32 bit patterns with the low half zero.
+// What is not finite: an infinity becomes (largest bf16, largest bf16, infinity), so that its products are what an infinity's are: inf
+// by nonzero and by infinite values, NaN by zero, with no inf - inf and no inf * 0 between the parts of a finite partner; a NaN
+// stays a NaN.  That takes two v_med3 a value, 3 % of a step (2048 tokens x 768 -> 3072, k = 256, fp32: 107 -> 110 us, and 112 with a
+// look at each stage's values instead), so FINITE leaves them out: an infinity then gives NaN wherever it is met, and a block
+// whose sums are not all finite runs its stages once more with them (104.4 us, against 103.4 without any of it in the same run).
+// A value that comes from a bf16 matrix has one part, and an infinite one gives NaN where its partner's lower parts are zero: the
+// products of bf16 layers do without the second run.
+template <bool FINITE> __device__ __forceinline__ void fg_split3(float v, uint32_t &h, uint32_t &m, uint32_t &l)
 {
-    h = __float_as_uint(v) & 0xffff0000u;
+    constexpr float top = 3.40282346638528859812e38f;
+    h = __float_as_uint(FINITE ? v : __builtin_amdgcn_fmed3f(v, -top, top)) & 0xffff0000u;
     const float r1 = v - __uint_as_float(h);
-    m = __float_as_uint(r1) & 0xffff0000u;
+    m = __float_as_uint(FINITE ? r1 : __builtin_amdgcn_fmed3f(r1, -top, top)) & 0xffff0000u;
     const float r2 = r1 - __uint_as_float(m);
     l = __float_as_uint(r2) & 0xffff0000u;
 }
@@ -240,7 +248,7 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
     // SPLIT: four of the thread's values into the planes, 8 bytes each, at element offset `at` of a plane.  Values that come from a
     // bf16 matrix are their own first part and the other two are zero: only the first plane is written (and read, see the kernel).
     __device__ __forceinline__ bool one_plane() const { return !HASHED && es == 2; }
-    template <bool ONE> __device__ __forceinline__ void put4(bf16_t *__restrict__ tile, int at, const f32x4 &v) const
+    template <bool ONE, bool FINITE> __device__ __forceinline__ void put4(bf16_t *__restrict__ tile, int at, const f32x4 &v) const
     {
         if (ONE) {
             *reinterpret_cast<uint2 *>(tile + at) = make_uint2((__float_as_uint(v[1]) & 0xffff0000u) | (__float_as_uint(v[0]) >> 16),
@@ -249,32 +257,32 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
         }
         uint32_t h[4], m[4], l[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) fg_split3(v[j], h[j], m[j], l[j]);
+        for (int j = 0; j < 4; ++j) fg_split3<FINITE>(v[j], h[j], m[j], l[j]);
         *reinterpret_cast<uint2 *>(tile + at) = make_uint2(h[1] | (h[0] >> 16), h[3] | (h[2] >> 16));
         *reinterpret_cast<uint2 *>(tile + PLANE + at) = make_uint2(m[1] | (m[0] >> 16), m[3] | (m[2] >> 16));
         *reinterpret_cast<uint2 *>(tile + 2 * PLANE + at) = make_uint2(l[1] | (l[0] >> 16), l[3] | (l[2] >> 16));
     }
-    template <bool ONE> __device__ __forceinline__ void store_split(bf16_t *__restrict__ tile) const
+    template <bool ONE, bool FINITE> __device__ __forceinline__ void store_split(bf16_t *__restrict__ tile) const
     {
         const int t = threadIdx.x & (FG_THREADS - 1);
         if (SRC == FG_KCONT) {
 #pragma unroll
             for (int h = 0; h < NV; ++h) {   // contraction values 4 kq .. 4 kq + 3 of a row
                 const int idx = h * FG_THREADS + t, row = idx >> 2, kq = idx & 3;
-                put4<ONE>(tile, ((kq >> 1) * ROWS + row) * 8 + (kq & 1) * 4, r[h]);
+                put4<ONE, FINITE>(tile, ((kq >> 1) * ROWS + row) * 8 + (kq & 1) * 4, r[h]);
             }
         } else if (SRC == FG_MCONT) {
 #pragma unroll
             for (int h = 0; h < NV; ++h) {   // four consecutive rows at one contraction value
                 const int idx = h * FG_THREADS + t, kk = idx / (ROWS / 4), r4 = (idx % (ROWS / 4)) * 4;
-                put4<ONE>(tile, kk * LDM + r4, r[h]);
+                put4<ONE, FINITE>(tile, kk * LDM + r4, r[h]);
             }
         } else {
             const int row = t % ROWS;
 #pragma unroll
             for (int h = 0; h < NV; ++h) {   // contraction values kk0 + 4 h .. + 3 of a row
                 const int kk = kk0 + 4 * h;
-                put4<ONE>(tile, ((kk >> 3) * ROWS + row) * 8 + (kk & 7), r[h]);
+                put4<ONE, FINITE>(tile, ((kk >> 3) * ROWS + row) * 8 + (kk & 7), r[h]);
             }
         }
     }
@@ -316,6 +324,7 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
     constexpr int UNITS = MI * NI * 2;   // a wave's accumulators in units of 8 registers: what the groups share out at the end
     constexpr int EXCHANGE = (G - 1) * UNITS * 4 * 512;
     __shared__ __align__(16) float lds_all[2 * STAGE * G > EXCHANGE ? 2 * STAGE * G : EXCHANGE];
+    __shared__ int not_finite;   // some thread's sum is an infinity or a NaN
     const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / FG_THREADS);
     float *lds = lds_all + group * 2 * STAGE;
     const int t = threadIdx.x & (FG_THREADS - 1), wave = t >> 6, lane = t & 63, r = lane & 31, g = lane >> 5, wm = wave >> 1, wn = wave & 1;
@@ -328,23 +337,18 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
     pa.init(p.a, p.lda, p.a_bytes, m0, p.M, k_begin, kend, p.seed, p.nsR, p.nsK, p.a_es);
     pb.init(p.b, p.ldb, p.b_bytes, n0, p.N, k_begin, kend, p.seed, p.nsR, p.nsK, p.b_es);
     f32x16 acc[MI][NI];
-#pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < NI; ++ni)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[mi][ni][e] = 0.0f;
-    pa.load(0);
-    pb.load(0);
+    if (threadIdx.x == 0) not_finite = 0;   // seen by everybody behind the first stage's barrier
     // The stage loop, once per number of planes of the two sides (known per launch, not per kernel: a side that comes from a
     // bf16 matrix has one plane), so that each copy is straight-line code between its barriers.
-    auto stages = [&](auto a_one, auto b_one) __attribute__((always_inline)) {
+    // ... and, for fp32 matrices, once more for sums that are not finite (fg_split3).
+    auto stages = [&](auto a_one, auto b_one, auto finite) __attribute__((always_inline)) {
         constexpr int AP = decltype(a_one)::value ? 1 : 3, BP = decltype(b_one)::value ? 1 : 3;
+        constexpr bool FINITE = decltype(finite)::value;
         for (int s = 0; s < nstage; ++s) {
             float *As = lds + (s & 1) * STAGE, *Bs = As + PA::TILE_BYTES / 4;
             if (SPLIT) {
-                pa.template store_split<AP == 1>(reinterpret_cast<bf16_t *>(As));
-                pb.template store_split<BP == 1>(reinterpret_cast<bf16_t *>(Bs));
+                pa.template store_split<AP == 1, PA::HASHED || FINITE>(reinterpret_cast<bf16_t *>(As));
+                pb.template store_split<BP == 1, PB::HASHED || FINITE>(reinterpret_cast<bf16_t *>(Bs));
             } else {
                 pa.store(As);
                 pb.store(Bs);
@@ -426,21 +430,47 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
     };
     typedef std::integral_constant<bool, true> One;
     typedef std::integral_constant<bool, false> Three;
-    if (!SPLIT || !ANY16) {   // ANY16: one of the matrices is bf16 (only then is the choice compiled in)
-        stages(Three{}, Three{});
-    } else {
-        const bool a1 = pa.one_plane(), b1 = pb.one_plane();
-        if (PA::HASHED || !a1) {
-            if (PB::HASHED || !b1) stages(Three{}, Three{});
-            else stages(Three{}, One{});
+    auto product = [&](auto finite) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[mi][ni][e] = 0.0f;
+        pa.load(0);
+        pb.load(0);
+        if (!SPLIT || !ANY16) {   // ANY16: one of the matrices is bf16 (only then is the choice compiled in)
+            stages(Three{}, Three{}, finite);
         } else {
-            if (PB::HASHED || !b1) stages(One{}, Three{});
-            else stages(One{}, One{});
+            const bool a1 = pa.one_plane(), b1 = pb.one_plane();
+            if (PA::HASHED || !a1) {
+                if (PB::HASHED || !b1) stages(Three{}, Three{}, finite);
+                else stages(Three{}, One{}, finite);
+            } else {
+                if (PB::HASHED || !b1) stages(One{}, Three{}, finite);
+                else stages(One{}, One{}, finite);
+            }
         }
+    };
+    product(std::true_type{});
+    bool again = false;
+    if (SPLIT && !ANY16) {
+        float zero = 0.0f;   // stays so as long as every sum is finite
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) zero = fmaf(acc[mi][ni][e], 0.0f, zero);
+        if (zero != 0.0f) not_finite = 1;
+        __syncthreads();   // also: the stage buffers are free
+        again = __builtin_amdgcn_readfirstlane(not_finite) != 0;
+        if (again) product(std::false_type{});
     }
     if constexpr (G > 1) {
+        const bool behind_barrier = !ANY16 && !again;
         // unit u (registers 8 (u % 2) .. of tile u / 2) is finished by group u * G / UNITS; the others hand theirs over
-        __syncthreads();   // the stage buffers are free
+        if (!behind_barrier) __syncthreads();   // the stage buffers are free
         auto slot = [&](int u, int from, int owner) { return lds_all + ((u * (G - 1) + (from < owner ? from : from - 1)) * 4 + wave) * 512 + lane; };
 #pragma unroll
         for (int u = 0; u < UNITS; ++u) {

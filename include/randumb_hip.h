@@ -385,9 +385,9 @@ int rdb_set_big_tiles(int mode);
 
 /* Tuning switch without a counterpart in the reference, for the products of fp32 layers (and of bf16 layers whose sizes are not
  * multiples of 8) and for the matrix-coef materialise products that run on the matrix cores.  mode 1 (default): every operand
- * value is split exactly into three bf16 parts (v = h + m + l, each the top 8 bits of what is left) on its way into LDS and a
+ * value is split exactly into three bf16 parts (v = h + m + l, each what is left rounded to the nearest) on its way into LDS and a
  * product runs as six bf16 matrix instructions (ah bh + ah bm + am bh + ah bl + al bh + am bm, fp32 accumulation): the terms
- * left out are below 2^-23 of a product, an fp32 multiplication's own rounding, and the 32 x 32 x 16 bf16 instruction does in
+ * left out are at most 1.01 * 2^-24 of a product, and the 32 x 32 x 16 bf16 instruction does in
  * 3/8 of the time what eight 32 x 32 x 2 fp32 ones do.  mode 0: fp32 matrix instructions.  Results agree to fp32 rounding;
  * infinities and NaNs in fp32 matrices come out as they do in mode 0, an infinity in a bf16 matrix (odd-sized bf16 layers) may
  * come out as NaN.  Process-wide; returns the previous mode. */

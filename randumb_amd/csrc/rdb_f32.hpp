@@ -52,25 +52,35 @@ struct FgParams {
     float *dot_part;            // with dotm: one value per block, in block order (x fastest, then y)
 };
 
-// fp32 products on the bf16 matrix cores.  v = h + m + l exactly, each part a bf16 (the top 8 bits of what is left: truncation,
-// so every difference is exact and the parts have v's sign).  A product a . b is then the sum of the nine products of the parts, each
-// exact in the matrix core's fp32 accumulation, of which the six largest are computed: ah bh + ah bm + am bh + ah bl + al bh + am bm.
-// The three left out, am bl + al bm + al bl, are less than 1.01 * 2^-21 |a b| (|m| < 2^-7 |v|, |l| < 2^-15 |v|; a = b = 1 + 2^-7 - 2^-23
-// comes to 2^-21.03), 2^-24.5 |a b| on average over normally distributed values.  Six bf16 matrix instructions of 32 x 32 x 16 do
-// the work of eight fp32 ones of 32 x 32 x 2 in 3/8 of the time.  The parts come back as fp32 bit patterns with the low half zero.
-// What is not finite: an infinity becomes (largest bf16, largest bf16, infinity), so that its products are what an infinity's are: inf
-// by nonzero and by infinite values, NaN by zero, with no inf - inf and no inf * 0 between the parts of a finite partner; a NaN
-// stays a NaN.  That takes two v_med3 a value, 3 % of a step (2048 tokens x 768 -> 3072, k = 256, fp32: 107 -> 110 us, and 112 with a
-// look at each stage's values instead), so FINITE leaves them out: an infinity then gives NaN wherever it is met, and a block
-// whose sums are not all finite runs its stages once more with them (104.4 us, against 103.4 without any of it in the same run).
-// A value that comes from a bf16 matrix has one part, and an infinite one gives NaN where its partner's lower parts are zero: the
-// products of bf16 layers do without the second run.
-template <bool FINITE> __device__ __forceinline__ void fg_split3(float v, uint32_t &h, uint32_t &m, uint32_t &l)
+// fp32 products on the bf16 matrix cores.  v = h + m + l exactly, each part a bf16: v rounded to the nearest, what is left rounded to
+// the nearest, and what is left of that (both differences are exact).  A product a . b is then the sum of the nine products of the
+// parts, each exact in the matrix core's fp32 accumulation, of which the six largest are computed: ah bh + ah bm + am bh + ah bl +
+// al bh + am bm.  The three left out, am bl + al bm + al bl, are of either sign and at most 1.01 * 2^-24 |a b|, what one rounding of the
+// product does (|m| <= 2^-8 |v|, |l| <= 2^-17 |v|), 2^-28 |a b| on average over normally distributed values.  (Parts cut off instead of
+// rounded leave out up to 1.01 * 2^-21 |a b|, always of the product's sign, and are no faster.)  Six bf16 matrix instructions of
+// 32 x 32 x 16 do the work of eight fp32 ones of 32 x 32 x 2 in 3/8 of the time.  fg_split3: two values at a time, the parts packed.
+__device__ __forceinline__ void fg_split3(float v0, float v1, uint32_t &h, uint32_t &m, uint32_t &l)
+{
+    h = f32x2_to_bf16x2(v0, v1);
+    v0 -= __uint_as_float(h << 16);
+    v1 -= __uint_as_float(h & 0xffff0000u);
+    m = f32x2_to_bf16x2(v0, v1);
+    l = f32x2_to_bf16x2(v0 - __uint_as_float(m << 16), v1 - __uint_as_float(m & 0xffff0000u));
+}
+// The same where a value may be infinite, or round to an infinity.  An infinity becomes (largest bf16, largest bf16, infinity), so
+// that its products are what an infinity's are: inf by nonzero and by infinite values, NaN by zero.  For that the parts are cut off
+// and not rounded: all of one sign, so that none of a product's terms overflows to the other side.  A NaN stays a NaN.  This takes two
+// v_med3 a value, 3 % of a step (2048 tokens x 768 -> 3072, k = 256, fp32: 107 -> 110 us, and 112 with a look at each stage's
+// values instead), so it is not done at first: an infinity then gives NaN wherever it is met, and a block whose sums are not all
+// finite runs its stages once more with it (104.4 us, against 103.4 without any of it in the same run).  A value that comes from
+// a bf16 matrix has one part, and an infinite one gives NaN where its partner's lower parts are zero: the products of bf16
+// layers do without the second run.
+__device__ __forceinline__ void fg_split3_any(float v, uint32_t &h, uint32_t &m, uint32_t &l)
 {
     constexpr float top = 3.40282346638528859812e38f;
-    h = __float_as_uint(FINITE ? v : __builtin_amdgcn_fmed3f(v, -top, top)) & 0xffff0000u;
+    h = __float_as_uint(__builtin_amdgcn_fmed3f(v, -top, top)) & 0xffff0000u;
     const float r1 = v - __uint_as_float(h);
-    m = __float_as_uint(FINITE ? r1 : __builtin_amdgcn_fmed3f(r1, -top, top)) & 0xffff0000u;
+    m = __float_as_uint(__builtin_amdgcn_fmed3f(r1, -top, top)) & 0xffff0000u;
     const float r2 = r1 - __uint_as_float(m);
     l = __float_as_uint(r2) & 0xffff0000u;
 }
@@ -255,12 +265,21 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
                                                                (__float_as_uint(v[3]) & 0xffff0000u) | (__float_as_uint(v[2]) >> 16));
             return;
         }
-        uint32_t h[4], m[4], l[4];
+        uint2 h, m, l;
+        if (FINITE) {
+            fg_split3(v[0], v[1], h.x, m.x, l.x);
+            fg_split3(v[2], v[3], h.y, m.y, l.y);
+        } else {
+            uint32_t p[4][3];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) fg_split3<FINITE>(v[j], h[j], m[j], l[j]);
-        *reinterpret_cast<uint2 *>(tile + at) = make_uint2(h[1] | (h[0] >> 16), h[3] | (h[2] >> 16));
-        *reinterpret_cast<uint2 *>(tile + PLANE + at) = make_uint2(m[1] | (m[0] >> 16), m[3] | (m[2] >> 16));
-        *reinterpret_cast<uint2 *>(tile + 2 * PLANE + at) = make_uint2(l[1] | (l[0] >> 16), l[3] | (l[2] >> 16));
+            for (int j = 0; j < 4; ++j) fg_split3_any(v[j], p[j][0], p[j][1], p[j][2]);
+            h = make_uint2(p[1][0] | (p[0][0] >> 16), p[3][0] | (p[2][0] >> 16));
+            m = make_uint2(p[1][1] | (p[0][1] >> 16), p[3][1] | (p[2][1] >> 16));
+            l = make_uint2(p[1][2] | (p[0][2] >> 16), p[3][2] | (p[2][2] >> 16));
+        }
+        *reinterpret_cast<uint2 *>(tile + at) = h;
+        *reinterpret_cast<uint2 *>(tile + PLANE + at) = m;
+        *reinterpret_cast<uint2 *>(tile + 2 * PLANE + at) = l;
     }
     template <bool ONE, bool FINITE> __device__ __forceinline__ void store_split(bf16_t *__restrict__ tile) const
     {
@@ -336,7 +355,13 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
     PB pb;
     pa.init(p.a, p.lda, p.a_bytes, m0, p.M, k_begin, kend, p.seed, p.nsR, p.nsK, p.a_es);
     pb.init(p.b, p.ldb, p.b_bytes, n0, p.N, k_begin, kend, p.seed, p.nsR, p.nsK, p.b_es);
-    f32x16 acc[MI][NI];
+    // The five smaller products of the parts in sums of their own (low), where registers allow it: the large sum is then rounded once a
+    // stage and not six times.  Distance from 64 bits, 13 layers of 32 to 1024 tokens with k <= 64, input gradient: 0.60 times that of
+    // fp32 multiplications and additions one after the other, as the vector-ALU kernels do them (1.01 times with one sum, 1.15 with
+    // one sum and parts cut off); outputs 0.68, coefficient gradients 0.46.  With it the 64-row kernels of one group would lose a
+    // quarter of their waves (2048 tokens x 768 -> 3072, k = 256: step 106.5 us against 104.4); their contractions are short.
+    constexpr bool APART = SPLIT && BM == 64 && G > 1 && !ANY16;
+    f32x16 acc[MI][NI], low[MI][NI];
     if (threadIdx.x == 0) not_finite = 0;   // seen by everybody behind the first stage's barrier
     // The stage loop, once per number of planes of the two sides (known per launch, not per kernel: a side that comes from a
     // bf16 matrix has one plane), so that each copy is straight-line code between its barriers.
@@ -379,13 +404,14 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
                     for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
                         for (int ni = 0; ni < NI; ++ni) {
-                            f32x16 c = acc[mi][ni];
+                            f32x16 c = APART ? low[mi][ni] : acc[mi][ni];
                             if constexpr (AP == 3 && BP == 3) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][1], fb[ni][1], c, 0, 0, 0);
                             if constexpr (AP == 3) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][2], fb[ni][0], c, 0, 0, 0);
                             if constexpr (BP == 3) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][0], fb[ni][2], c, 0, 0, 0);
                             if constexpr (AP == 3) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][1], fb[ni][0], c, 0, 0, 0);
                             if constexpr (BP == 3) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][0], fb[ni][1], c, 0, 0, 0);
-                            acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][0], fb[ni][0], c, 0, 0, 0);
+                            if (APART) low[mi][ni] = c;
+                            acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi][0], fb[ni][0], APART ? acc[mi][ni] : c, 0, 0, 0);
                             constexpr int GROUPS = MI * NI;
                             const int grp = mi * NI + ni;
                             if (PB::HASHED && more) {
@@ -436,7 +462,7 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
 #pragma unroll
             for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) acc[mi][ni][e] = 0.0f;
+                for (int e = 0; e < 16; ++e) acc[mi][ni][e] = low[mi][ni][e] = 0.0f;
         pa.load(0);
         pb.load(0);
         if (!SPLIT || !ANY16) {   // ANY16: one of the matrices is bf16 (only then is the choice compiled in)
@@ -450,6 +476,14 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
                 if (PB::HASHED || !b1) stages(One{}, Three{}, finite);
                 else stages(One{}, One{}, finite);
             }
+        }
+        if (APART) {
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+                for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[mi][ni][e] += low[mi][ni][e];
         }
     };
     product(std::true_type{});

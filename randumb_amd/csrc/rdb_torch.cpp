@@ -320,9 +320,8 @@ class OneCallLinear : public Function<OneCallLinear> {
                           const OptTensor &bias_scale, int64_t bias_seed, const Layer &l)
     {
         const Bias b{bias, bias_scale, bias_seed};
-        ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, l.sO, l.sI, (int64_t)l.seed, scale_bias ? 1 : 0};
+        ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, l.sO, l.sI, (int64_t)l.seed, scale_bias ? 1 : 0, coefs.size(0), coefs.size(-1)};
         ctx->saved_data["bias"] = b.meta();
-        ctx->saved_data["coefs"] = coefs.sizes().vec();
         const Tensor x = act(x0);
         const bool same = x.scalar_type() == coefs.scalar_type() && readable(coefs.scalar_type()) && (!scale_bias || scale_bias->numel() == 1);
         const rdb_linear_desc d = desc(x, l, coefs);
@@ -348,7 +347,7 @@ class OneCallLinear : public Function<OneCallLinear> {
         const Layer l{m[0], m[1], m[2], m[3], (uint32_t)m[4]};
         const bool has_sb = m[5] != 0;
         constexpr const char *who = "linear (backward)";
-        restored(who, coefs, grads[0], ctx->saved_data["coefs"].toIntVector());
+        restored(who, coefs, grads[0], at::IntArrayRef(&m[6], coefs.dim() == 1 ? 1 : 2));
         if (x.defined()) restored(who, x, grads[0], {grads[0].size(0), l.in_f});
         if (has_sb) restored(who, sb, grads[0], sb.sizes());
         const at::AutoGradMode no_grad(false);

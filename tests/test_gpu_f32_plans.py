@@ -38,3 +38,23 @@ def test_materialise_and_adjoint(rows, k, row_len):
     noise = ops.sq5_gen_2d(row_len, k, 3).double().cpu()
     assert _rel(hip.materialize_fwd(c.cuda(), (rows, row_len), (row_len, 1), 3, None, False), c.double() @ noise.t()) < 2e-6
     assert _rel(hip.materialize_bwd(d.cuda(), k, 3, rows), d.double() @ noise) < 2e-6
+
+
+@pytest.mark.parametrize("tokens,in_f,out_f,k", [(51, 205, 468, 43), (137, 764, 161, 27), (66, 2253, 280, 28), (44, 226, 251, 19), (725, 246, 906, 44),
+                                                 (300, 512, 1024, 64)])
+def test_few_token_products_are_no_further_from_64_bits_than_fp32_ones(tokens, in_f, out_f, k):
+    """Layers of few tokens and coefficients, which the vector ALU's fp32 kernels may run as well, against the same two products in
+    the library's fp32.  Its sums are cut into pieces too, so neither is systematically ahead: 1.1 covers that."""
+    from randumb_amd import hip
+
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x, dy, c = (torch.randn(*s, device="cuda", generator=g) for s in ((tokens, in_f), (tokens, out_f), (out_f, k)))
+    N = hip.sq5_fill_2d(in_f, k, 7)
+    off = lambda a, b: float((a.double() - b).norm() / b.norm())
+    y, dx = hip.linear_fwd(x, c, in_f, out_f, in_f, 1, 7), hip.linear_bwd_dx(dy, c, in_f, out_f, in_f, 1, 7)
+    dc, _ = hip.linear_bwd_dcoef(dy, x, k, out_f, in_f, out_f, in_f, 1, 7)
+    z, t = x.double() @ N.double(), dy.double() @ c.double()
+    for name, got, plain, exact in (("y", y, (x @ N) @ c.t(), z @ c.double().t()), ("dx", dx, (dy @ c) @ N.t(), t @ N.double().t()),
+                                    ("dcoef", dc, dy.t() @ (x @ N), dy.double().t() @ z)):
+        print(f"  {name}: {off(got, exact):.2e}, in fp32 {off(plain, exact):.2e}", flush=True)
+        assert off(got, exact) <= 1.1 * off(plain, exact), name

@@ -418,6 +418,11 @@ int rdb_sync_giveups(uint32_t *count, void *stream);
  * throughout, the counter above grows by the number of blocks, every kernel ends normally. */
 int rdb_selftest_sync_giveup(void *y, int64_t ldy, void *scratch, int64_t scratch_bytes, const void *coef,
                              const rdb_linear_desc *desc, int polls, void *stream);
+/* Test hook: rdb_linear_project_fwd (bf16, without a bias) whose multiplying blocks wait for `polls` polls only: each of them
+ * either computes its share of y or, its wait having run out, leaves NaN there; what projecting blocks store in y's rows
+ * on the way does not stay in either case. */
+int rdb_selftest_hasty_wait(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *desc, int polls,
+                            void *stream);
 
 /* ------------------------------------------------------------------------------------------ around the linears of a block
  * The parts of a transformer block between its pseudorandom linears, in bf16 with fp32 arithmetic, each as one pass (or one

@@ -68,6 +68,7 @@ EXPORTS = [
     "rdb_sync_giveups_async",
     "rdb_sync_giveups",
     "rdb_selftest_sync_giveup",
+    "rdb_selftest_hasty_wait",
     "rdb_rms_norm_fwd",
     "rdb_rms_norm_bwd",
     "rdb_relu_square",
@@ -215,6 +216,8 @@ def load() -> ctypes.CDLL:
     L.rdb_sync_giveups.restype = ci
     L.rdb_selftest_sync_giveup.argtypes = [vp, i64, vp, i64, vp, dp, ci, vp]
     L.rdb_selftest_sync_giveup.restype = ci
+    L.rdb_selftest_hasty_wait.argtypes = [vp, i64, vp, vp, i64, vp, dp, ci, vp]
+    L.rdb_selftest_hasty_wait.restype = ci
     for name in ("rdb_sq5_fill_2d", "rdb_sq5_fill_1d", "rdb_materialize_fwd", "rdb_materialize_bwd", "rdb_scale_bias_bwd",
                  "rdb_embed_fwd", "rdb_embed_bwd", "rdb_linear_fwd", "rdb_linear_bwd_dx", "rdb_linear_bwd_dx_dscale", "rdb_linear_rbias_fwd",
                  "rdb_linear_rbias_fwd_ws", "rdb_linear_project_fwd_rbias", "rdb_linear_rbias_bwd", "rdb_linear_bwd_dcoef",

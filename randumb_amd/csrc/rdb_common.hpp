@@ -196,6 +196,19 @@ __device__ __forceinline__ bool await_tags(const unsigned long long *slots, int 
     return false;
 }
 
+// Where a producer may still be on its way to memory that a consumer owns (sums on the way in its output's rows): a consumer that has
+// given up leaves the launch's tag in a word of theirs before it poisons its output, and the producer looks at the word
+// once its own stores are in memory.  Either the producer sees it and poisons what it wrote, or its stores came first.
+__device__ __forceinline__ void mark_gone(unsigned int *word, unsigned long long tag)
+{
+    if ((threadIdx.x & 63) == 0) __hip_atomic_store(word, (unsigned int)tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(0);
+}
+__device__ __forceinline__ bool is_gone(const unsigned int *word, unsigned long long tag)
+{
+    return __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned int)tag;
+}
+
 // The same wave calls this once its wait has succeeded.  A launch recorded in a graph runs again with the tag it was recorded
 // with, so the slots must not still hold it then: every consumer of the n slots counts itself in `counter`, and the last of
 // the `consumers` (all of them are past their wait by then) clears the slots.  The counter is set to zero by one of the

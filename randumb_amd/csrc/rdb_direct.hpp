@@ -23,13 +23,13 @@ __host__ __device__ inline int64_t frag_index(int64_t row, int64_t kk, int64_t k
 
 // Where the pieces of a layer's projection state lie in the caller's buffer (a pure function of the layer's sizes).
 //   header : 256 bytes; word 0 = 1 when the transposed coefficients below are present; word 1 != 0: a launch that waits for its
-//            own earlier blocks gave up waiting (never seen; the results of that launch are then undefined)
+//            own earlier blocks gave up waiting (never seen; what those blocks stood for is then NaN)
 //   zf     : z = x . N^T for the forward product: fragment order [tokens32 / 32][kpad / 16], rows = tokens
 //   ztf    : z transposed, fragment order, rows = coefficients: [kpad / 32][tokens64 / 16]   (operand of dC = dy^T . z)
 //   ctf    : C transposed, fragment order, rows = coefficients: [kpad / 32][out64 / 16]      (operand of t = dy . C)
 //   sync   : per 256 tokens, one 64-bit slot per projection tile (32 coefficients) with the tag of the launch that wrote the tile
-//            last, and one counter of the blocks that have consumed them: for the forward launch whose later blocks consume
-//            what its earlier blocks project
+//            last, and one counter of the blocks that have consumed them (beside it, the low half of the tag once a consumer has
+//            given up): for the forward launch whose later blocks consume what its earlier blocks project
 // kpad, tokens64, out64: rounded up to 64; tokens32: to 32.
 struct ProjLayout {
     bool ok, fits_regs;   // fits_regs: k <= 256, the forward product keeps a token's whole contraction in registers

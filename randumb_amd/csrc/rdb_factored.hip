@@ -39,7 +39,8 @@ struct ZParams {
     int tiles_m, tiles_t;
     uint32_t seed;
     unsigned long long *sync;   // NULL, or slots [tiles_t][tiles_m + 1]: a block sets its slot to sync_tag when its tile is in memory;
-                                // slot tiles_m of a token tile counts its consumers and is cleared by the block of coefficient tile 0
+                                // slot tiles_m of a token tile counts its consumers (low half, cleared by the block of coefficient tile 0)
+                                // and holds the low half of the tag once one of them has given up (high half)
     unsigned long long sync_tag;
     // The contraction is added up in `ranges` ranges of range_stages stages of 64 features, range by range, whoever computes them.
     // part == NULL: every block runs its tile's ranges one after the other.  Otherwise the grid holds a block per tile and range,
@@ -233,11 +234,27 @@ template <bool RANGES> __device__ __forceinline__ void z_block(const ZParams &p,
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v), rs_p, (int)at(my_range, jq), 0, SCOPE_DEVICE);
             }
             publish_tag(tags + my_range, p.sync_tag);
+            if (p.sync) {   // the rows are a multiplying block's: has it given up, and filled them with NaN before these sums came?
+                volatile int *gone = reinterpret_cast<volatile int *>(smem_raw);
+                if (t == 0) {
+                    __builtin_amdgcn_s_waitcnt(0);   // the tag too is in memory
+                    *gone = is_gone(reinterpret_cast<unsigned int *>(p.sync + (int64_t)(w / p.tiles_m) * (p.tiles_m + 1) + p.tiles_m) + 1, p.sync_tag);
+                }
+                __syncthreads();
+                if (*gone) {
+                    const i32x4 nan8 = {0x7fc07fc0, 0x7fc07fc0, 0x7fc07fc0, 0x7fc07fc0};
+#pragma unroll
+                    for (int jq = 0; jq < 4; ++jq) __builtin_amdgcn_raw_buffer_store_b128(nan8, rs_p, (int)at(my_range, jq), 0, SCOPE_DEVICE);
+                    if (t == 0) __hip_atomic_store(tags + my_range, 0x7fc07fc07fc07fc0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
             return;
         }
         volatile int *verdict = reinterpret_cast<volatile int *>(smem_raw);
         if (wave == 0) {
             const bool there = await_tags(tags, others, p.sync_tag, p.sync_wait);
+            if (!there && p.sync)
+                mark_gone(reinterpret_cast<unsigned int *>(p.sync + (int64_t)(w / p.tiles_m) * (p.tiles_m + 1) + p.tiles_m) + 1, p.sync_tag);
             if (lane == 0) *verdict = there ? 1 : 0;
         }
         __syncthreads();
@@ -564,8 +581,9 @@ template <int KG, bool BIAS> static int launch_zy(const ZYParams &p, int y_items
 
 // state <- projection of x (with the transposed coefficients if with_ct), y <- forward product, in one launch when the
 // contraction of a token fits in registers (k <= 256), otherwise in two.
+// polls: how long its multiplying blocks wait; fewer than SYNC_SPIN_LIMIT in a self-test only.
 int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, bool with_ct, const void *bias,
-                       const rdb_linear_desc *d, int num_cus, hipStream_t s)
+                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls)
 {
     ZYParams p;
     if (!fill_z_params(p.z, state, x, ldx, with_ct ? coef : nullptr, d)) return RDB_E_UNSUPPORTED;
@@ -584,7 +602,7 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
     p.y.sync_tag = p.z.sync_tag;
     p.y.sync_n = p.z.tiles_m;
     p.y.sync_wait.err = reinterpret_cast<unsigned int *>(state) + 1;
-    p.y.sync_wait.polls = SYNC_SPIN_LIMIT;
+    p.y.sync_wait.polls = polls;
     if (int rc = sync_giveups_ptr(&p.y.sync_wait.giveups)) return rc;
     int rc;
     const bool spread = spread_ranges(p.z, state, y, ldy, d, &rc);
@@ -697,7 +715,7 @@ int linear_fwd_factored(void *y, int64_t ldy, const void *x, int64_t ldx, const 
     if (d->tokens * ldx >= (1ll << 29) || ldx % 8 || ldy % 8 || !aligned16(x) || !aligned16(coef) || !aligned16(y) || !aligned16(workspace))
         return RDB_E_UNSUPPORTED;
     if (((uintptr_t)bias & 7) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
-    return linear_project_fwd(y, ldy, workspace, x, ldx, coef, false, bias, d, num_cus, s);
+    return linear_project_fwd(y, ldy, workspace, x, ldx, coef, false, bias, d, num_cus, s, SYNC_SPIN_LIMIT);
 }
 
 // dC = dy^T . (x . N^T) with the projection state in the workspace; dcoef must have been zeroed on the same stream.

@@ -287,7 +287,7 @@ int linear_fwd_strip(void *y, int64_t ldy, const void *x, int64_t ldx, const voi
 int64_t linear_projection_bytes(const rdb_linear_desc *d);
 int linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, hipStream_t s);
 int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, bool with_ct, const void *bias,
-                       const rdb_linear_desc *d, int num_cus, hipStream_t s);
+                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls = SYNC_SPIN_LIMIT);
 int linear_fwd_projected(void *y, int64_t ldy, const void *z, const void *coef, const void *bias, const rdb_linear_desc *d, int num_cus,
                          hipStream_t s);
 int linear_dcoef_projected(float *dcoef, const void *dy, int64_t lddy, const void *z, const rdb_linear_desc *d, int num_cus, hipStream_t s);
@@ -1333,6 +1333,21 @@ extern "C" int rdb_selftest_sync_giveup(void *y, int64_t ldy, void *scratch, int
     if (rc == RDB_E_UNSUPPORTED)
         return set_error(RDB_E_UNSUPPORTED, "rdb_selftest_sync_giveup: needs a layer whose forward has a one-launch form (bf16 matrix-coef, k <= 256, "
                                             "or fp32 matrix-coef, k <= 64, in_f <= 8192) and its scratch (projection state / forward workspace)");
+    return rc;
+}
+
+extern "C" int rdb_selftest_hasty_wait(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, int polls,
+                                       void *stream)
+{
+    ChunkPlan pl;
+    int rc = check_projected("rdb_selftest_hasty_wait", d, &pl);
+    if (rc) return rc;
+    if (!y || !state || !x || !coef) return set_error(RDB_E_NULL, "rdb_selftest_hasty_wait: y, state, x or coef is NULL");
+    if (polls < 1 || polls > SYNC_SPIN_LIMIT) return set_error(RDB_E_SHAPE, "rdb_selftest_hasty_wait: polls must be 1 .. %d", SYNC_SPIN_LIMIT);
+    if (ldx < d->in_f || ldy < d->out_f) return set_error(RDB_E_SHAPE, "rdb_selftest_hasty_wait: leading dimension smaller than the row");
+    rc = pl.nchunks != 1 ? RDB_E_UNSUPPORTED
+                         : linear_project_fwd(y, ldy, state, x, ldx, coef, true, nullptr, d, num_compute_units(), (hipStream_t)stream, polls);
+    if (rc == RDB_E_UNSUPPORTED) return set_error(rc, "rdb_selftest_hasty_wait: needs a bf16 layer of one chunk of tokens that rdb_linear_project_fwd takes");
     return rc;
 }
 

@@ -232,6 +232,7 @@ __device__ __forceinline__ void stationary_block(const StParams &p, unsigned cha
             if (wave == 0) {
                 unsigned long long *slots = p.sync + (int64_t)(w / p.splits) * (p.sync_n + 1);
                 const bool there = await_tags(slots, p.sync_n, p.sync_tag, p.sync_wait);
+                if (!there) mark_gone(reinterpret_cast<unsigned int *>(slots + p.sync_n) + 1, p.sync_tag);
                 if (there) release_tags(slots, p.sync_n, reinterpret_cast<unsigned int *>(slots + p.sync_n), p.splits);
                 if (b.lane == 0) *verdict = there ? 1 : 0;
             }

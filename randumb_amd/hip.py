@@ -183,6 +183,20 @@ def selftest_sync_giveup(y: torch.Tensor, scratch: torch.Tensor, coef: torch.Ten
     _lib.check(rc, "rdb_selftest_sync_giveup")
 
 
+def selftest_hasty_wait(x: torch.Tensor, coef: torch.Tensor, seed: int, polls: int = 1) -> torch.Tensor:
+    """Test hook: ``y`` of :func:`linear_project_fwd` (bf16) with a wait of ``polls`` polls in its multiplying blocks: NaN where one of
+    them gave up."""
+    _need_gpu("selftest_hasty_wait", x, coef)
+    x, coef = _act(x), coef.contiguous()
+    pl = _plan(x.shape[0], x.shape[1], coef.shape[0], coef.shape[1], seed, x.dtype)
+    state = torch.empty(max(pl.state_bytes, 1), dtype=torch.uint8, device=x.device)
+    y = torch.empty((x.shape[0], coef.shape[0]), dtype=x.dtype, device=x.device)
+    with _on(x.device):
+        rc = _lib.load().rdb_selftest_hasty_wait(_p(y), y.stride(0), _p(state), _p(x), x.stride(0), _p(coef), pl.ref, int(polls), _stream(x.device))
+    _lib.check(rc, "rdb_selftest_hasty_wait")
+    return y
+
+
 # ------------------------------------------------------------------------------------------------ probes
 def sq5_fill_2d(N: int, M: int, seed: int, device="cuda") -> torch.Tensor:
     """Noise matrix ``(N, M)``, ``out[n, m] = noise(PRIME*n + m)``  (RandumbTensor.py:101-105)."""

@@ -121,3 +121,29 @@ def test_transposed_coefficients_from_blocks_of_their_own(T, in_f, out_f, k, one
     assert torch.equal(y, hip.linear_fwd_projected(plain, c, in_f, 5))
     for dx, dc in results[:2]:
         assert torch.equal(dx, results[2][0]) and torch.equal(dc, results[2][1])
+
+
+@pytest.mark.parametrize("T,in_f,out_f,k", [(300, 4096, 4096, 64), (97, 8192, 2048, 64), (512, 8192, 1024, 32), (2000, 4096, 4096, 256)])
+def test_sums_on_the_way_do_not_stay_in_the_rows_of_a_block_that_gave_up(hip, T, in_f, out_f, k):
+    """Multiplying blocks that look once and give up leave NaN; projecting blocks that are still at work then put their sums into
+    the same rows, and have to take them back.  Every value of y is its own or NaN, in whole blocks of tokens."""
+    from randumb_amd import _lib
+
+    print(f"case hasty wait T={T} in={in_f} out={out_f} k={k}", flush=True)
+    x, C = _inputs(T, in_f, out_f, k)
+    hip.sync_check()
+    want, _ = hip.linear_project_fwd(x, C, 5)
+    seen = 0
+    try:
+        for _ in range(3):
+            y = hip.selftest_hasty_wait(x, C, 5, polls=1)
+            poisoned = y.isnan()
+            seen += int(poisoned.any())
+            assert torch.equal(y[~poisoned], want[~poisoned])
+        assert seen, "no block gave up"
+        with pytest.raises(_lib.RandumbHipError, match="gave up"):
+            hip.sync_check()
+    finally:
+        hip.set_one_launch(1)
+    assert torch.equal(hip.linear_project_fwd(x, C, 5)[0], want)
+    hip.sync_check()

@@ -197,3 +197,77 @@ def test_blocks_that_share_their_normalisation():
         # the embedding's gradient is summed with atomics by the library
         assert all(torch.equal(a, b) or float((a - b).float().norm() / b.float().norm()) < 4e-3 for a, b in zip(results[0], other))
         assert sum(torch.equal(a, b) for a, b in zip(results[0], other)) >= len(other) - 1
+
+
+def _loss_in_64_bits(model, idx, target):
+    """RT_GPT.forward in fp64 on leaves that are the model's parameters: (loss, gradients in the parameters' order).  The angles of
+    the rotary embedding are the bf16 ones the model has: they are what it computes, not how exactly."""
+    from randumb_amd import hip
+
+    leaves = {n: p.detach().double().requires_grad_() for n, p in model.named_parameters() if "scale_bias" not in n}
+
+    def linear(x, name, layer):
+        N = hip.sq5_fill_2d(layer.in_features, layer.weight_coef.shape[1], layer.seed[0]).double()
+        return (x @ N) @ leaves[name + ".weight_coef"].t()
+
+    def norm(x):
+        return F.rms_norm(x, (x.size(-1),), eps=EPS)
+
+    x = norm(leaves["wte.weight"][idx])
+    B, T, D = x.shape
+    for i, block in enumerate(model.h):
+        H = block.attn.n_head
+        freqs = torch.outer(torch.arange(T, device=x.device), block.attn.rotary.inv_freq)
+        cos, sin = freqs.cos().double()[None, :, None, :], freqs.sin().double()[None, :, None, :]
+
+        def rot(t):
+            t1, t2 = norm(t).chunk(2, dim=3)
+            return torch.cat((t1 * cos + t2 * sin, t2 * cos - t1 * sin), 3).transpose(1, 2)
+
+        q, k, v = linear(norm(x), f"h.{i}.attn.c_qkv", block.attn.c_qkv).view(B, T, 3, H, 64).unbind(2)
+        s = (rot(q) @ rot(k).transpose(-1, -2).contiguous()) / 8.0
+        s = s.masked_fill(torch.ones(T, T, dtype=torch.bool, device=x.device).triu(1), -math.inf)
+        y = (s.softmax(-1) @ v.transpose(1, 2).contiguous()).transpose(1, 2).reshape(B, T, D)
+        x = x + linear(y, f"h.{i}.attn.c_proj", block.attn.c_proj)
+        x = x + linear(F.relu(linear(norm(x), f"h.{i}.mlp.c_fc", block.mlp.c_fc)).square(), f"h.{i}.mlp.c_proj", block.mlp.c_proj)
+    loss = F.cross_entropy((norm(x) @ leaves["lm_head.weight"].t()).view(-1, leaves["lm_head.weight"].shape[0]), target.view(-1))
+    return loss.detach(), dict(zip(leaves, torch.autograd.grad(loss, list(leaves.values()))))
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2])
+def test_the_fused_model_is_no_further_from_64_bits_than_the_stock_one(ext, monkeypatch, seed):
+    """A bf16 training step with the fused kernels and with the stock operators around the same linears, each against the same
+    model in fp64.  Their roundings are different ones, so single gradients may differ either way (a quarter); over all of them
+    the fused step must not be further off (5 % for chance)."""
+    from randumb_amd import gpt
+
+    torch.manual_seed(seed)
+    with torch.device("cuda"):
+        model = gpt.RT_GPT(gpt.RT_GPTConfig(int_dim_gen=iter([64] * 16), seed_gen=iter(range(16)), vocab_size=1024, n_layer=4, n_head=4, n_embd=256)).bfloat16()
+        ids = torch.randint(0, 1024, (3, 193))
+    with torch.no_grad():
+        model.lm_head.weight.normal_(0.0, 0.02)
+        for m in model.modules():
+            if isinstance(m, gpt.RT_CastedLinear):
+                m.weight_coef.mul_(2.0)
+    idx, target = ids[:, :-1].contiguous(), ids[:, 1:].contiguous()
+    exact_loss, exact = _loss_in_64_bits(model, idx, target)
+    off = {}
+    for fused in (True, False):
+        if not fused:
+            monkeypatch.setattr(gpt, "_fused", lambda x: None)
+        model.zero_grad(set_to_none=True)
+        loss = model(idx, target)
+        loss.backward()
+        off[fused] = {n: rel(p.grad, exact[n]) for n, p in model.named_parameters() if p.grad is not None and n in exact}
+        off[fused]["loss"] = abs(float(loss.detach().double() - exact_loss) / float(exact_loss))
+    grads = [n for n in off[True] if n != "loss"]
+    assert len(grads) == 2 + 16
+    ratios = {n: off[True][n] / off[False][n] for n in grads}
+    mean = math.exp(sum(math.log(r) for r in ratios.values()) / len(ratios))
+    print(f"  fused against stock, distance from 64 bits: gradients {mean:.3f} times, at most {max(ratios.values()):.3f}; "
+          f"loss {off[True]['loss']:.2e} and {off[False]['loss']:.2e}; a gradient is off by {max(off[True][n] for n in grads):.1e}", flush=True)
+    assert mean <= 1.05 and max(ratios.values()) <= 1.25, ratios
+    # One number, so chance alone decides which loss is nearer.  A logit (0.3 typically) is off by some 1.4e-2 of itself, as the gradients
+    # are; over 576 rows the mean is off by 4e-3 / 24 = 1.8e-4, 2.5e-5 of a loss of 6.9.  Four times that.
+    assert off[True]["loss"] <= 1e-4 and off[False]["loss"] <= 1e-4

@@ -17,8 +17,9 @@
 //
 // Measured at 8 sequences x 12 heads x 1024 tokens, us: prep 13.5, forward 29.9, dq 44.6, dk / dv 55.8 (144 in all; the stock
 // operators they replace: attention 81 forward, 267 backward, normalisation and rotation some 450).  13 GFLOP forward and 45
-// backward: the forward pass is bound by the exponentials on the vector ALU (16 a lane for 16 matrix instructions) rather than
-// by the matrix cores.
+// backward.  No pipe is full (SQ counters, shares of a compute unit's time): matrix cores 24 to 29 %, vector ALU 42 to 48 % (25 % of the
+// forward pass in exponentials, 16 a lane for 16 matrix instructions), LDS 32 to 41 % without bank conflicts; two waves a SIMD and a
+// barrier per 64 rows put them one after the other.  The preparing kernel is the vector ALU's (81 %).
 #include "rdb_gemm.hpp"
 
 namespace rdb {

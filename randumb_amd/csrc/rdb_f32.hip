@@ -485,7 +485,7 @@ int materialize_mat_f32(float *out, const void *coef, int coef_dtype, int64_t co
                        0, 0, 0, 0, seed, (uint32_t)row_len, 1u, (const float *)scale_bias, nullptr, 0, nullptr};
         q.a_es = fg_es(coef_dtype);
         q.scale_bf16 = coef_dtype == RDB_BF16;
-            return fg_launch<FG_KCONT, FG_NOISE_I>(q, num_cus, s, "f32_gemm_kernel (W = C . N)");
+        return fg_launch<FG_KCONT, FG_NOISE_I>(q, num_cus, s, "f32_gemm_kernel (W = C . N)");
     }
     // W^T[i, o]: rows = i hashed, columns = o from C; the random bias at index o * row_len + i
     FgProduct q = {nullptr, 0, 0, C, k, coef_rows * k, out, coef_rows, nullptr, row_len, coef_rows, k,

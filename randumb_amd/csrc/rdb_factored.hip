@@ -386,8 +386,9 @@ template <int KG, bool BIAS> __global__ __launch_bounds__(ST_THREADS, 1) void fa
 }
 
 // Projection and forward product in one launch: blocks 0 .. z_grid - 1 project (z_block), the next c_blocks transpose C, the others multiply
-// (stationary_block; z_grid and c_blocks are multiples of 8, so that all kinds keep their numbering over the dies) and wait, tile by tile, for the tags of the projection blocks that feed them.  A multiplying block
-// starts on a compute unit the moment a projecting block leaves it: no drain of the whole chip, no second launch in between.
+// (stationary_block; z_grid and c_blocks are multiples of 8, so that all kinds keep their numbering over the dies) and wait, tile
+// by tile, for the tags of the projection blocks that feed them.  A multiplying block starts on a compute unit the moment a
+// projecting block leaves it: no drain of the whole chip, no second launch in between.
 struct ZYParams {
     ZParams z;
     StParams y;

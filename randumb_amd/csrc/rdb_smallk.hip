@@ -144,7 +144,8 @@ template <int KMAX, typename E, bool HASH> __device__ __forceinline__ void small
         const int cc = c < cols ? c : cols - 1;
 #pragma unroll
         for (int m = 0; m < KB; ++m) {
-            if (m % 16 == 0 && m >= k) break;   // uniform  // branch-free: a column from k on reads a valid address and becomes 0
+            if (m % 16 == 0 && m >= k) break;   // uniform
+            // branch-free: a column from k on reads a valid address and becomes 0
             const float v = HASH ? sq5_unit(sq5_tail(sq5_first((uint32_t)cc, (uint32_t)m, seed))) : elem<E>::load(coef + (int64_t)cc * k + ((m < k) ? m : k - 1));
             b0[m] = (m < k) ? v : 0.0f;
         }

@@ -385,7 +385,10 @@ class _ProjectedFunction(torch.autograd.Function):
 
 def _coef_form(t) -> Optional[tuple]:
     """``(coefs, scale or None, seed)`` of a contiguous vector-coef tensor in its coefficients' dtype, as the extension module takes
-    a pseudorandom bias or weight (autograd then reaches the coefficients there); None for other pseudorandom tensors."""
+    a pseudorandom bias or weight (autograd then reaches the coefficients there, past the tensor itself); None for other
+    pseudorandom tensors, and for one whose own gradient somebody waits for."""
+    if t.retains_grad or t._backward_hooks:
+        return None
     if t.coef_rows or t.dtype != t._coef.dtype or type(t._coef) not in _PLAIN or not t.is_contiguous():
         return None
     c, sb = t._coef, t.scale_bias if t.fused_bias else None

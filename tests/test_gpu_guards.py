@@ -233,3 +233,25 @@ def test_rows_farther_apart_than_one_launch_addresses(form, sliced):
     got = [y.detach(), *torch.autograd.grad(y, wanted, spread(dy) if sliced == "dy" else dy)]
     for a, b in zip(got, ref):
         assert torch.equal(a, b)
+
+
+# ------------------------------------------------------------------------------------------------ gradients of the pseudorandom tensors themselves
+@pytest.mark.parametrize("how", ["retain_grad", "register_hook"])
+@pytest.mark.parametrize("form,which", [("vector_fp32", "weight"), ("vector_fp32", "bias"), ("kept_bf16", "bias"), ("projected_bf16", "bias"), ("one_call_fp32", "bias")])
+def test_somebody_who_waits_for_a_tensors_own_gradient_gets_it(form, which, how):
+    layer, x = _layer(form)
+    wanted = [x, layer.weight_coef, layer.bias_coef]
+    dy = torch.randn(x.shape[0], layer.out_features, device="cuda").to(x.dtype)
+    ref = torch.autograd.grad(layer(x), wanted, dy)
+    t, seen = getattr(layer, which), []
+    if how == "retain_grad":
+        t.retain_grad()
+    else:
+        t.register_hook(lambda g: seen.append(g.detach().clone()))
+    layer(x).backward(dy)
+    grad = t.grad if how == "retain_grad" else seen[0]
+    want = (dy.double().t() @ x.detach().double()) if which == "weight" else dy.double().sum(0)
+    assert grad.shape == t.shape
+    assert float((grad.double() - want).norm()) <= (1e-5 if x.dtype == torch.float32 else 1e-2) * float(want.norm())
+    for p, r in zip(wanted, ref):
+        assert float((p.grad.double() - r.double()).norm()) <= (1e-5 if x.dtype == torch.float32 else 2e-2) * float(r.double().norm())

@@ -538,12 +538,12 @@ class CoefValues : public Function<CoefValues> {
     }
 };
 
-// out [M x N] = A . B^T (+ bias); A [M x K], B [N x K], or stored transposed (across).  fp32: the library's own product; bf16: torch's
-Tensor product(const Tensor &a, bool a_across, const Tensor &b, bool b_across, const Tensor &bias)
+// out [M x N], contiguous, = A . B^T (+ bias); A [M x K], B [N x K], or stored transposed (across).  fp32: the library's own product;
+// bf16: torch's.  out is the caller's, because what an autograd function returns must not be a view (in-place changes of it are refused)
+const Tensor &product(const Tensor &out, const Tensor &a, bool a_across, const Tensor &b, bool b_across, const Tensor &bias)
 {
     const int64_t M = a.size(a_across ? 1 : 0), K = a.size(a_across ? 0 : 1), N = b.size(b_across ? 1 : 0);
     if (a.scalar_type() == at::kFloat) {
-        Tensor out = at::empty({M, N}, a.options());
         const int64_t need = rdb_product_f32_workspace_bytes(M, N, K);
         const Tensor ws = bytes(need, a);
         const int rc = rdb_product_f32(out.data_ptr<float>(), a.data_ptr<float>(), a.stride(0), a_across, b.data_ptr<float>(), b.stride(0), b_across,
@@ -554,7 +554,10 @@ Tensor product(const Tensor &a, bool a_across, const Tensor &b, bool b_across, c
         }
     }
     const Tensor l = a_across ? a.t() : a, r = b_across ? b : b.t();
-    return bias.defined() ? at::addmm(bias, l, r) : at::mm(l, r);
+    Tensor to = out.view({M, N});
+    if (bias.defined()) at::addmm_out(to, bias, l, r);
+    else at::mm_out(to, l, r);
+    return out;
 }
 
 // y = x.W^T (+ b) with W and b vector-coef tensors: W is formed (k hashed values per element), multiplied as a dense matrix, and
@@ -584,7 +587,7 @@ class VectorLinear : public Function<VectorLinear> {
     {
         auto sizes = x0.sizes().vec();
         sizes.back() = l.out_f;
-        return product(act(x0.reshape({-1, l.in_f})), false, W, false, b.values(l.out_f, x0.scalar_type())).view(sizes);
+        return product(at::empty(sizes, x0.options()), act(x0.reshape({-1, l.in_f})), false, W, false, b.values(l.out_f, x0.scalar_type()));
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
@@ -621,10 +624,11 @@ class VectorLinear : public Function<VectorLinear> {
             const bool kept = saved[3].defined();
             if (kept) restored(who, restored_values(who, saved[3], dy, x0.scalar_type(), l.out_f * l.in_f), dy, {l.out_f, l.in_f});
             const Tensor W = kept ? saved[3] : coef_values(coef, scale, l.out_f * l.in_f, l.seed).view({l.out_f, l.in_f});
-            dx = product(dy, false, W, true, Tensor()).view(x0.sizes());
+            dx = product(at::empty(x0.sizes(), dy.options()), dy, false, W, true, Tensor());
         }
         if (want_c || want_s) {
-            const auto g = coef_grads(product(dy, true, act(x0.reshape({-1, l.in_f})), true, Tensor()), coef.numel(), l.seed, want_c, want_s);
+            const Tensor dW = product(at::empty({l.out_f, l.in_f}, dy.options()), dy, true, act(x0.reshape({-1, l.in_f})), true, Tensor());
+            const auto g = coef_grads(dW, coef.numel(), l.seed, want_c, want_s);
             if (want_c) dc = g.first.to(coef.scalar_type());
             if (want_s) ds = g.second.to((at::ScalarType)m[3]);
         }

@@ -255,3 +255,20 @@ def test_somebody_who_waits_for_a_tensors_own_gradient_gets_it(form, which, how)
     assert float((grad.double() - want).norm()) <= (1e-5 if x.dtype == torch.float32 else 1e-2) * float(want.norm())
     for p, r in zip(wanted, ref):
         assert float((p.grad.double() - r.double()).norm()) <= (1e-5 if x.dtype == torch.float32 else 2e-2) * float(r.double().norm())
+
+
+# ------------------------------------------------------------------------------------------------ outputs that are changed in place
+@pytest.mark.parametrize("dims", [2, 3])
+@pytest.mark.parametrize("form", FORMS + ["vector_bf16"])
+def test_a_layers_output_may_be_changed_in_place(form, dims):
+    """As that of F.linear: relu_(layer(x)), and its gradient."""
+    layer, x = _layer(form.replace("vector_bf16", "vector_fp32"))
+    if form == "vector_bf16":
+        layer, x = layer.bfloat16(), x.detach().bfloat16().requires_grad_()
+    if dims == 3:
+        x = x.detach().unsqueeze(0).requires_grad_()
+    (want,) = torch.autograd.grad(torch.relu(layer(x)).sum(), x)
+    y = layer(x)
+    assert not y._is_view() or dims == 3
+    (got,) = torch.autograd.grad(y.relu_().sum(), x)
+    assert torch.equal(got, want)

@@ -95,6 +95,9 @@ class SyncWatch:
         self.seen = 0
         self.pending = None
 
+    def _capturing(self) -> bool:
+        return self._event_factory is None and torch.cuda.is_current_stream_capturing()
+
     def _library(self):
         return self._lib if self._lib is not None else _lib.load()
 
@@ -125,9 +128,13 @@ class SyncWatch:
         """Called by the entry points that may run a one-launch kernel (or once per several of their calls); never waits for the
         device."""
         before, self.calls = self.calls, self.calls + calls
+        due = self.pending is None and before // self.every != self.calls // self.every
+        if (due or self.pending is not None) and self._capturing():
+            return   # a recorded copy and event would tell nothing, and asking an event ends a capture: looked at by later calls
         if self.pending is not None and self.pending.query():
             self._judge()
-        if self.pending is None and before // self.every != self.calls // self.every:
+            due = before // self.every != self.calls // self.every
+        if due:
             self._enqueue(stream)
 
     def check(self, stream) -> None:

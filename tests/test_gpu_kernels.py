@@ -652,3 +652,37 @@ def test_projected_path_random_shapes(hip, oracle):
         assert rel_l2(cpu(y), want_y) < BF16_TOL, case
         assert rel_l2(cpu(dx), want_dx) < BF16_TOL, case
         assert rel_l2(cpu(dc), want_dc) < BF16_TOL, case
+
+
+def test_more_calls_than_the_watch_waits_for_recorded_into_one_graph(hip):
+    """200 calls of a layer in one capture: the watch counts them and does not look.  Replayed with other inputs and eager work between."""
+    T, in_f, out_f, k = 64, 256, 256, 32
+    x, _, coef = _inputs(T, in_f, out_f, k, True, torch.bfloat16, 3)
+    xg, cg = x.cuda(), coef.cuda()
+    from randumb_amd import ops
+
+    def many(v):
+        for _ in range(200):
+            v = ops.linear(v, cg, in_f, out_f, in_f, 1, 3, None, None)
+            v = v / v.float().abs().amax().clamp_min(1e-6).to(v.dtype)
+        return v
+
+    with torch.no_grad():
+        inputs = [xg, xg.flip(0).contiguous(), (xg * 0.5).contiguous()]
+        want = [many(v).clone() for v in inputs]
+        static = inputs[0].clone()
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            many(static)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = many(static)
+        for v, w in zip(inputs, want):
+            static.copy_(v)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, w)
+            many(v)   # eager calls between the replays look at the counter
+    hip.sync_check()

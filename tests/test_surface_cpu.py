@@ -118,6 +118,49 @@ def test_sync_watch_host_logic():
         w.check(None)
 
 
+def test_nothing_is_looked_at_while_a_graph_is_recorded(monkeypatch):
+    """A copy and an event recorded into a graph say nothing of the work, and asking an event during a capture is an error: calls
+    are counted then, and the first one behind a multiple outside of the capture looks."""
+    from randumb_amd import hip
+
+    host = torch.zeros(1, dtype=torch.int32)
+
+    class Lib:
+        copies = 0
+
+        def rdb_sync_giveups_async(self, dst, stream):
+            self.copies += 1
+            return 0
+
+    class Event:
+        asked = 0
+
+        def record(self):
+            pass
+
+        def query(self):
+            Event.asked += 1
+            return True
+
+    lib = Lib()
+    w = hip.SyncWatch(lib=lib, host_word=host, event_factory=Event, every=4)
+    capturing = [True]
+    monkeypatch.setattr(w, "_capturing", lambda: capturing[0])
+    for _ in range(9):
+        w.tick(None)
+    assert w.calls == 9 and lib.copies == 0 and w.pending is None
+    capturing[0] = False
+    for _ in range(3):
+        w.tick(None)
+    assert lib.copies == 1 and w.pending is not None
+    capturing[0] = True
+    w.tick(None, 8)
+    assert Event.asked == 0 and w.pending is not None
+    capturing[0] = False
+    w.tick(None)
+    assert Event.asked == 1 and w.pending is None
+
+
 def test_explicit_look_sees_what_came_after_a_pending_one():
     """A copy of the counter that tick has asked for says nothing of the work enqueued after it: check takes one of its own."""
     from randumb_amd import _lib, hip

@@ -713,6 +713,12 @@ void need_bf16(const char *who, const Tensor &t)
 {
     if (!t.is_cuda() || t.scalar_type() != at::kBFloat16) fail(PyExc_ValueError, std::string(who) + " needs bf16 tensors on the GPU");
 }
+// Contiguous from a 16-byte boundary on: the kernels read 8 and 16 bytes at a time, and a contiguous slice may begin anywhere.
+Tensor dense(const Tensor &t)
+{
+    const Tensor c = t.contiguous();
+    return (uintptr_t)c.data_ptr() % 16 ? c.clone() : c;
+}
 int64_t row_count(const Tensor &x) { return x.size(-1) ? x.numel() / x.size(-1) : 0; }
 
 // A gradient asked for under create_graph is computed by the stock operators, from the inputs as they were given.
@@ -722,7 +728,7 @@ class RmsNorm : public Function<RmsNorm> {
   public:
     static Tensor forward(AutogradContext *ctx, const Tensor &x0, double eps)
     {
-        const Tensor x = x0.contiguous();
+        const Tensor x = dense(x0);
         const c10::OptionalDeviceGuard guard(x.device());
         Tensor y = at::empty_like(x), rstd = at::empty({row_count(x)}, x.options().dtype(at::kFloat));
         check(rdb_rms_norm_fwd(y.data_ptr(), nullptr, rstd.data_ptr<float>(), x.data_ptr(), nullptr, row_count(x), x.size(-1), (float)eps, stream_of(x)),
@@ -741,7 +747,7 @@ class RmsNorm : public Function<RmsNorm> {
             const double eps = ctx->saved_data["eps"].toDouble();
             return {stock_gradient([&](const variable_list &in) { return variable_list{stock(in[0], eps)}; }, {saved[0]}, {grads[0]})[0], Tensor()};
         }
-        const Tensor x = saved[0].contiguous(), dy = grads[0].contiguous();
+        const Tensor x = dense(saved[0]), dy = dense(grads[0]);
         restored_values(who, x, dy, at::kBFloat16, dy.numel());
         restored_values(who, saved[1], dy, at::kFloat, row_count(dy));
         const c10::OptionalDeviceGuard guard(x.device());
@@ -757,7 +763,7 @@ class AddRmsNorm : public Function<AddRmsNorm> {
   public:
     static variable_list forward(AutogradContext *ctx, const Tensor &x0, const Tensor &delta0, double eps)
     {
-        const Tensor x = x0.contiguous(), delta = delta0.contiguous();
+        const Tensor x = dense(x0), delta = dense(delta0);
         const c10::OptionalDeviceGuard guard(x.device());
         Tensor y = at::empty_like(x), sum = at::empty_like(x), rstd = at::empty({row_count(x)}, x.options().dtype(at::kFloat));
         check(rdb_rms_norm_fwd(y.data_ptr(), sum.data_ptr(), rstd.data_ptr<float>(), x.data_ptr(), delta.data_ptr(), row_count(x), x.size(-1), (float)eps,
@@ -781,7 +787,7 @@ class AddRmsNorm : public Function<AddRmsNorm> {
             if (d.defined() && grads[0].defined()) d = d + grads[0];
             return {d, d, Tensor()};
         }
-        const Tensor dy = grads[1].contiguous(), dsum = grads[0].defined() ? grads[0].contiguous() : Tensor();
+        const Tensor dy = dense(grads[1]), dsum = grads[0].defined() ? dense(grads[0]) : Tensor();
         restored_values(who, x, dy, at::kBFloat16, dy.numel());
         restored_values(who, saved[1], dy, at::kFloat, row_count(dy));
         const c10::OptionalDeviceGuard guard(x.device());
@@ -796,7 +802,7 @@ class ReluSquare : public Function<ReluSquare> {
   public:
     static Tensor forward(AutogradContext *ctx, const Tensor &x0)
     {
-        const Tensor x = x0.contiguous();
+        const Tensor x = dense(x0);
         const c10::OptionalDeviceGuard guard(x.device());
         Tensor y = at::empty_like(x);
         check(rdb_relu_square(y.data_ptr(), x.data_ptr(), nullptr, x.numel(), stream_of(x)), "rdb_relu_square");
@@ -810,7 +816,7 @@ class ReluSquare : public Function<ReluSquare> {
         restored(who, x0, grads[0], grads[0].sizes());
         if (at::GradMode::is_enabled())
             return stock_gradient([](const variable_list &in) { return variable_list{at::relu(in[0]).square()}; }, {x0}, {grads[0]});
-        const Tensor x = x0.contiguous(), dy = grads[0].contiguous();
+        const Tensor x = dense(x0), dy = dense(grads[0]);
         restored_values(who, x, dy, at::kBFloat16, dy.numel());
         const c10::OptionalDeviceGuard guard(x.device());
         Tensor dx = at::empty_like(x);
@@ -824,7 +830,7 @@ class CrossEntropy : public Function<CrossEntropy> {
   public:
     static Tensor forward(AutogradContext *ctx, const Tensor &logits0, const Tensor &target0, int64_t ignore)
     {
-        const Tensor logits = logits0.contiguous(), target = target0.contiguous();
+        const Tensor logits = dense(logits0), target = target0.contiguous();
         const c10::OptionalDeviceGuard guard(logits.device());
         const int64_t rows = logits.size(0);
         Tensor loss = at::empty({}, logits.options().dtype(at::kFloat)), scratch = at::empty({2 * rows + 1}, loss.options());
@@ -848,7 +854,7 @@ class CrossEntropy : public Function<CrossEntropy> {
             };
             return {stock_gradient(loss, {saved[0]}, {grads[0]})[0], Tensor(), Tensor()};
         }
-        const Tensor logits = saved[0].contiguous(), dloss = grads[0].to(at::kFloat).contiguous();
+        const Tensor logits = dense(saved[0]), dloss = grads[0].to(at::kFloat).contiguous();
         restored_values(who, logits, dloss, at::kBFloat16, m[0] * m[1]);
         restored_values(who, saved[2], dloss, at::kFloat, 2 * m[0] + 1);
         const c10::OptionalDeviceGuard guard(logits.device());
@@ -865,7 +871,7 @@ class CausalAttention : public Function<CausalAttention> {
   public:
     static Tensor forward(AutogradContext *ctx, const Tensor &qkv0, const Tensor &inv_freq0, int64_t heads, double eps)
     {
-        const Tensor qkv = qkv0.contiguous(), inv_freq = native(inv_freq0);
+        const Tensor qkv = dense(qkv0), inv_freq = native(inv_freq0);
         const c10::OptionalDeviceGuard guard(qkv.device());
         const int64_t B = qkv.size(0), T = qkv.size(1);
         Tensor y = at::empty({B, T, heads * 64}, qkv.options()), q = at::empty({B * heads, T, 64}, qkv.options()), k = at::empty_like(q);
@@ -886,7 +892,7 @@ class CausalAttention : public Function<CausalAttention> {
     static Tensor gradient(AutogradContext *ctx, const variable_list &saved, const Tensor &grad)
     {
         const at::AutoGradMode no_grad(false);
-        const Tensor &qkv = saved[0], dy = grad.contiguous();
+        const Tensor &qkv = saved[0], dy = dense(grad);
         constexpr const char *who = "causal_attention (backward)";
         const int64_t B = dy.size(0), T = dy.size(1), heads = ctx->saved_data["heads"].toInt();
         restored(who, restored_values(who, qkv, dy, at::kBFloat16, 3 * dy.numel()), dy, {B, T, 3 * heads * 64});

@@ -61,6 +61,32 @@ def test_relu_square_is_the_stock_chain_bit_for_bit(ext, n):
     assert torch.equal(ga.nan_to_num(7), gb.nan_to_num(7))
 
 
+@pytest.mark.parametrize("offset", [1, 2, 4, 6])
+@pytest.mark.parametrize("op", ["rms_norm", "add_rms_norm", "relu_square", "cross_entropy", "causal_attention"])
+def test_slices_that_begin_between_the_boundaries_of_wide_loads(ext, op, offset):
+    """Contiguous inputs and gradients `offset` values behind a 16-byte boundary: the results of aligned ones."""
+    g = torch.Generator(device="cuda").manual_seed(offset)
+
+    def at(t, off):
+        buf = torch.empty(t.numel() + 16, device="cuda", dtype=t.dtype)
+        return buf[off : off + t.numel()].view(t.shape).copy_(t)
+
+    x, d = bf16(g, 2, 9, 192), bf16(g, 2, 9, 192)
+    t = torch.randint(0, 192, (18,), device="cuda", generator=g)
+    inv = torch.ones(32, device="cuda")
+    f = {"rms_norm": lambda a, b: ext.rms_norm(a, EPS), "add_rms_norm": lambda a, b: ext.add_rms_norm(a, b, EPS)[1], "relu_square": lambda a, b: ext.relu_square(a),
+         "cross_entropy": lambda a, b: ext.cross_entropy(a.view(18, 192), t, -100), "causal_attention": lambda a, b: ext.causal_attention(a, inv, 1, EPS)}[op]
+    out = []
+    for off in (0, offset):
+        a, b = at(x, off).requires_grad_(), at(d, off)
+        y = f(a, b)
+        dy = at(torch.arange(y.numel(), device="cuda").remainder(7).to(y.dtype).view(y.shape) - 3, off if y.dim() else 0)
+        out.append([y.detach(), torch.autograd.grad(y, a, dy)[0]])
+    assert a.data_ptr() % 16 != 0
+    for p, q in zip(*out):
+        assert torch.equal(p, q)
+
+
 def test_relu_square_with_gradients_that_are_not_finite(ext):
     """Where x <= 0 the stock operators pass nothing on, an infinite gradient included."""
     v = torch.tensor([-2.0, -0.0, 0.0, 1.5, math.inf, -math.inf, math.nan], device="cuda").bfloat16()

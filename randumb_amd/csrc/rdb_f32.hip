@@ -11,7 +11,7 @@
 // N[m, i] = noise(PRIME*i + m) is hashed into the pipeline's LDS tiles and never stored; W = C . N is never formed.  All
 // five products run on one kernel template that differs in where its two operands come from (a row-major matrix read along
 // or across its rows, or the hash).  Operands, intermediate matrices and sums are fp32 in memory and in the accumulators.  (bf16 layers whose sizes keep them off
-// the bf16 kernels, which want multiples of 8, run here too: bf16 matrices are read value by value and widened, z and t stay
+// the bf16 kernels, which want multiples of 8, run here too: a bf16 value is its own first part, z and t stay
 // fp32, y and dx are rounded to bf16 once.)
 // With scale_bias (W = C . N + s . R, R[o, i] = noise1d(o*in_f + i), full rank: src/rten_cpp/RandumbTensor.py:286-289) the
 // random-bias share is one more product with R as the hashed operand, added on top:  y += s * x . R^T,  dx += s * dy . R,  and
@@ -85,7 +85,7 @@ int set_f32_split_mode(int mode)
 }
 
 // The shapes these kernels take: matrix-coef fp32, matrices below 2^31 bytes.  Extents, leading dimensions and pointers that are
-// multiples of 4 elements / 16 bytes get the kernels that read 16 bytes at a time, everything else the value-by-value ones.
+// multiples of 4 elements / 16 bytes get the kernels that read aligned pieces, everything else those that read four values at any address.
 static bool fg_ok(const rdb_linear_desc *d)
 {
     const bool f32 = d->act_dtype == RDB_F32 && d->coef_dtype == RDB_F32, b16 = d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16;

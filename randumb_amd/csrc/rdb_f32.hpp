@@ -42,7 +42,7 @@ struct FgParams {
     int kchunk;          // contraction values per split (a multiple of FG_BK); K when there is one split
     int64_t a_bytes, b_bytes;   // extent of the matrices, for the bounds check of the loads (< 2^31)
     uint32_t seed;
-    int a_es, b_es;             // bytes per element of the A and B matrices: 4, or 2 (bf16; only the value-by-value kernels)
+    int a_es, b_es;             // bytes per element of the A and B matrices: 4, or 2 (bf16)
     int out_bf16;               // out, bias and dotm are bf16 (the activations' dtype)
     int scale_bf16;             // scale is bf16 (the coefficients' dtype)
     uint32_t nsR, nsK;          // FG_NOISE_1D: index steps per row and per contraction value
@@ -89,17 +89,26 @@ __device__ __forceinline__ void fg_split3_any(float v, uint32_t &h, uint32_t &m,
 // them into a tile.  Rows past `rows` and contraction values past `kend` are zeros.
 // VEC: the matrix is read in pieces of four values (16 bytes of fp32, 8 bytes of bf16; 16-byte aligned base, leading dimension a
 // multiple of 4, and the extent that runs along a piece a multiple of 4, so that a piece lies inside or outside as a whole);
-// otherwise four values at a time at any address where all four exist, value by value at the edges.
+// otherwise four values at a time at any address, see load4u.
 // SPLIT: the tile goes to LDS as three bf16 planes (see fg_split3): planes of [2 halves of the stage's 16 contraction values]
 // [rows][8] for the sources read along the contraction (a lane's MFMA operand is 16 consecutive bytes), of [16][rows + 32] for
 // FG_MCONT (read back with the LDS transpose read).  The noise sources then give a thread consecutive contraction values.
-template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
+// ES: bytes per element of the matrix, 4 or 2 (bf16).  Known to the compiler, because a load whose width is chosen by a branch has to
+// be widened inside the branch, and so waited for where it is requested: every stage of a product with a bf16 matrix cost a memory
+// latency (4097 tokens x 1001 -> 999 in bf16, k = 100: t = dy . C 21.0 -> 11.2 us, dC 17.5 -> 14.3, z 17.1 -> 15.7, step 91.8 -> 80.9).
+// bf16 values stay as they are until they reach their one plane.  0: known per launch (es; not SPLIT).
+template <int ROWS, int SRC, bool VEC, bool SPLIT = false, int ES = 4> struct FgOperand {
+    static_assert(SPLIT ? ES == 4 || ES == 2 : ES == 0, "the fp32 matrix instructions' kernels learn the element's size at run time");
     static constexpr int LD = ROWS + 4, TILE = FG_BK * LD, NV = ROWS * FG_BK / FG_THREADS / 4;   // float4 per thread and stage
     static_assert(NV >= 1, "a stage is at least one float4 per thread");
+    static constexpr bool HASHED = SRC == FG_NOISE_M || SRC == FG_NOISE_I || SRC == FG_NOISE_1D;
+    static constexpr bool ONE = ES == 2 && !HASHED;   // values that are their own first part: only the first plane is written and read
     static constexpr int LDM = ROWS + 32;                                            // FG_MCONT plane: elements per contraction value
     static constexpr int PLANE = SRC == FG_MCONT ? FG_BK * LDM : 2 * ROWS * 8;       // bf16 elements of one plane
-    static constexpr int TILE_BYTES = SPLIT ? 3 * PLANE * 2 : TILE * 4;
+    static constexpr int TILE_BYTES = SPLIT ? (ONE ? 1 : 3) * PLANE * 2 : TILE * 4;
     static constexpr int KPT = NV * 4;                                               // SPLIT, noise: consecutive contraction values per thread
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef std::conditional_t<ONE, u32x2, f32x4> Piece;   // four values as they are on their way to LDS
     __amdgpu_buffer_rsrc_t rs;
     uint32_t off[NV];   // byte offset of the thread's pieces at stage 0
     bool ok[NV];        // ... and whether the piece's (first) row exists
@@ -107,49 +116,102 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
     uint32_t first;     // noise: first-round value of the thread's first element at stage 0
     int kk0, kend, k_begin, row_ok;
     int rows_left[NV];  // FG_MCONT without VEC: how many of the piece's four rows exist
-    f32x4 r[NV];
+    bool edge, tiny;    // without VEC, the same for the whole block: some piece is not whole; some row has fewer than four values
+    Piece r[NV];
 
     uint32_t inc;       // noise: first-round step per contraction value
     const char *base;   // the matrix, for load4u
-    int es;             // bytes per element of the matrix (2: bf16)
-    __device__ __forceinline__ float load1(uint32_t o, bool in, int j) const
+    int es;             // bytes per element of the matrix
+    // VEC: four consecutive elements at byte offset o, zeros when outside
+    __device__ __forceinline__ Piece load4(uint32_t o, bool in) const
     {
-        if (es == 2) {
-            const unsigned short h = __builtin_amdgcn_raw_buffer_load_b16(rs, in ? (int)(o + 2 * j) : (int)FG_OOB, 0, 0);
-            return bf16_to_f32(h);
+        if constexpr (ONE) {
+            return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, in ? (int)o : (int)FG_OOB, 0, 0));
+        } else {
+            if (ES == 0 && es == 2) {
+                const u32x2 h = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, in ? (int)o : (int)FG_OOB, 0, 0));
+                return f32x4{__uint_as_float(h[0] << 16), __uint_as_float(h[0] & 0xffff0000u), __uint_as_float(h[1] << 16), __uint_as_float(h[1] & 0xffff0000u)};
+            }
+            return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, in ? (int)o : (int)FG_OOB, 0, 0));
         }
-        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, in ? (int)(o + 4 * j) : (int)FG_OOB, 0, 0));
     }
-    // VEC: four consecutive elements at byte offset o (fp32: 16 bytes; bf16: 8 bytes, widened), zeros when outside
-    __device__ __forceinline__ f32x4 load4(uint32_t o, bool in) const
+    // not VEC: four consecutive elements at any element's address (the hardware takes loads of 8 and 16 bytes at any address; 4097 tokens
+    // x 1001 features in bf16, k = 100: z = x . N^T 20.8 us with a load per value, 14.4 us with these).  Where only the first n of
+    // the four exist, the last four that do are loaded, from 4 - n elements before, and moved down by whole() when the piece
+    // is stored: no branch that would have to wait for its loads.
+    __device__ __forceinline__ Piece load4u(uint32_t o) const
     {
-        if (es == 2) {
-            const f32x2 h = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, in ? (int)o : (int)FG_OOB, 0, 0));
-            const uint32_t lo = __float_as_uint(h[0]), hi = __float_as_uint(h[1]);
-            return f32x4{__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u), __uint_as_float(hi << 16), __uint_as_float(hi & 0xffff0000u)};
-        }
-        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, in ? (int)o : (int)FG_OOB, 0, 0));
-    }
-    // not VEC: four consecutive elements that all exist, at any element's address (the hardware takes loads of 8 and 16 bytes at
-    // any address; 4097 tokens x 1001 features in bf16, k = 100: z = x . N^T 20.8 us with a load per value, 14.4 us with these)
-    __device__ __forceinline__ f32x4 load4u(uint32_t o) const
-    {
-        if (es == 2) {
-            typedef uint32_t pair_any __attribute__((ext_vector_type(2), aligned(2)));
-            const pair_any h = *reinterpret_cast<const pair_any *>(base + o);
-            return f32x4{__uint_as_float(h[0] << 16), __uint_as_float(h[0] & 0xffff0000u), __uint_as_float(h[1] << 16), __uint_as_float(h[1] & 0xffff0000u)};
-        }
+        typedef uint32_t pair_any __attribute__((ext_vector_type(2), aligned(2)));
         typedef float quad_any __attribute__((ext_vector_type(4), aligned(4)));
-        const quad_any v = *reinterpret_cast<const quad_any *>(base + o);
-        return f32x4{v[0], v[1], v[2], v[3]};
+        if constexpr (ONE) {
+            const pair_any h = *reinterpret_cast<const pair_any *>(base + o);
+            return u32x2{h[0], h[1]};
+        } else {
+            if (ES == 0 && es == 2) {
+                const pair_any h = *reinterpret_cast<const pair_any *>(base + o);
+                return f32x4{__uint_as_float(h[0] << 16), __uint_as_float(h[0] & 0xffff0000u), __uint_as_float(h[1] << 16), __uint_as_float(h[1] & 0xffff0000u)};
+            }
+            const quad_any v = *reinterpret_cast<const quad_any *>(base + o);
+            return f32x4{v[0], v[1], v[2], v[3]};
+        }
     }
-    __device__ __forceinline__ void init(const float *src, int64_t ld, int64_t bytes, int row0, int rows, int k_begin_, int kend_, uint32_t seed,
+    // the first n (any number) of four elements, one by one: rows of fewer than four values
+    __device__ __forceinline__ Piece load_first(uint32_t o, int n) const
+    {
+        Piece v = {};
+        const bool b16 = ES == 2 || (ES == 0 && es == 2);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int at = j < n ? (int)(o + (b16 ? 2 : 4) * j) : (int)FG_OOB;
+            if (b16) {
+                const uint32_t h = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(rs, at, 0, 0);
+                if constexpr (ONE) v[j / 2] |= h << (16 * (j & 1));
+                else v[j] = __uint_as_float(h << 16);
+            } else if constexpr (!ONE) {
+                v[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0));
+            }
+        }
+        return v;
+    }
+    // not VEC: how many of the values of piece h of a stage exist (any number: none when below 1, all when above 3)
+    __device__ __forceinline__ int existing(int stage, int h) const
+    {
+        const int kk = k_begin + stage * FG_BK + kk0;
+        if (SRC == FG_KCONT) return ok[h] ? kend - kk : 0;
+        return ok[h] && kk + h * (FG_THREADS / (ROWS / 4)) < kend ? rows_left[h] : 0;
+    }
+    __device__ __forceinline__ Piece request(int stage, int h) const
+    {
+        const uint32_t o = off[h] + (uint32_t)stage * step;
+        const int n = existing(stage, h);
+        if (tiny) return load_first(o, n);
+        const uint32_t e = ES ? (uint32_t)ES : (uint32_t)es;
+        return load4u(n >= 4 ? o : n > 0 ? o - (uint32_t)(4 - n) * e : 0u);
+    }
+    // ... and the piece as it belongs: the values that exist first, zeros behind them
+    __device__ __forceinline__ Piece whole(int stage, int h) const
+    {
+        Piece v = r[h];
+        if (VEC || HASHED || !edge) return v;
+        const int n = existing(stage, h);
+        if (tiny || n >= 4) return v;
+        if constexpr (ONE) {
+            const uint64_t w = n > 0 ? (((uint64_t)v[1] << 32) | v[0]) >> (16 * (4 - n)) : 0;
+            v = u32x2{(uint32_t)w, (uint32_t)(w >> 32)};
+        } else {
+            if (n <= 2) v = f32x4{v[2], v[3], 0.0f, 0.0f};
+            if (n & 1) v = f32x4{v[1], v[2], v[3], 0.0f};
+            if (n <= 0) v = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        return v;
+    }
+    __device__ __forceinline__ void init(const float *src, int64_t ld, int64_t bytes, int row0, int rows, int K, int k_begin_, int kend_, int nstage, uint32_t seed,
                                          uint32_t sR, uint32_t sK, int es_)
     {
         const int t = threadIdx.x & (FG_THREADS - 1);
         k_begin = k_begin_;
         kend = kend_;
-        es = es_;
+        es = ES ? ES : es_;
         base = reinterpret_cast<const char *>(src);
         if (SRC == FG_KCONT) {
             rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(src), 0, (int)bytes, 0x00020000);
@@ -161,6 +223,8 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
                 off[h] = ok[h] ? (uint32_t)(((int64_t)(row0 + row) * ld + k_begin + kq * 4) * es) : 0u;
             }
             kk0 = (t & 3) * 4;
+            tiny = K < 4;
+            edge = row0 + ROWS > rows || kend_ - k_begin_ != nstage * FG_BK;
         } else if (SRC == FG_MCONT) {
             rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(src), 0, (int)bytes, 0x00020000);
             step = (uint32_t)(FG_BK * ld * es);
@@ -172,6 +236,8 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
                 rows_left[h] = rows - (row0 + r4);
             }
             kk0 = t / (ROWS / 4);
+            tiny = rows < 4;
+            edge = row0 + ROWS > rows || kend_ - k_begin_ != nstage * FG_BK;
         } else {
             const int row = t % ROWS;
             kk0 = SPLIT ? (t / ROWS) * KPT : t / ROWS;
@@ -188,65 +254,47 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
     }
     __device__ __forceinline__ void load(int stage)
     {
-        if (SRC == FG_KCONT) {
-            // a thread's four values are consecutive contraction values
-            const int kk = k_begin + stage * FG_BK + kk0;
-#pragma unroll
-            for (int h = 0; h < NV; ++h) {
-                const uint32_t o = off[h] + (uint32_t)stage * step;
-                if (VEC) {   // all inside or all outside
-                    r[h] = load4(o, ok[h] && kk < kend);
-                } else if (ok[h] && kk + 4 <= kend) {
-                    r[h] = load4u(o);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) r[h][j] = load1(o, ok[h] && kk + j < kend, j);
-                }
-            }
-        } else if (SRC == FG_MCONT) {
-#pragma unroll
-            for (int h = 0; h < NV; ++h) {
-                const bool in = ok[h] && k_begin + stage * FG_BK + kk0 + h * (FG_THREADS / (ROWS / 4)) < kend;
-                const uint32_t o = off[h] + (uint32_t)stage * step;
-                if (VEC) {
-                    r[h] = load4(o, in);
-                } else if (in && rows_left[h] >= 4) {
-                    r[h] = load4u(o);
-                } else {   // a thread's four values are consecutive rows: rows_left of them exist
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) r[h][j] = load1(o, in && j < rows_left[h], j);
-                }
-            }
-        } else {
+        if constexpr (HASHED) {
 #pragma unroll
             for (int j = 0; j < NV * 4; ++j) hash_piece(stage, j);
+        } else if constexpr (VEC) {   // all inside or all outside
+            // a thread's four values are consecutive contraction values (FG_KCONT) or consecutive rows (FG_MCONT)
+            const int kk = k_begin + stage * FG_BK + kk0;
+#pragma unroll
+            for (int h = 0; h < NV; ++h)
+                r[h] = load4(off[h] + (uint32_t)stage * step, ok[h] && kk + (SRC == FG_MCONT ? h * (FG_THREADS / (ROWS / 4)) : 0) < kend);
+        } else {
+#pragma unroll
+            for (int h = 0; h < NV; ++h) r[h] = request(stage, h);
         }
     }
     // Noise sources: element j of the thread's NV * 4 values of a stage (contraction value kk0 + j * (FG_THREADS / ROWS), one add
     // apart in the first round).  The main loop calls this between the matrix instructions of the stage before.
-    static constexpr bool HASHED = SRC == FG_NOISE_M || SRC == FG_NOISE_I || SRC == FG_NOISE_1D;
     __device__ __forceinline__ void hash_piece(int stage, int j)
     {
-        constexpr int KSTEP = SPLIT ? 1 : FG_THREADS / ROWS;
-        const uint32_t f = first + (uint32_t)(stage * FG_BK + j * KSTEP) * inc;
-        const bool in = row_ok && k_begin + stage * FG_BK + kk0 + j * KSTEP < kend;
-        r[j >> 2][j & 3] = in ? sq5_unit(sq5_tail(f)) : 0.0f;
+        if constexpr (HASHED) {
+            constexpr int KSTEP = SPLIT ? 1 : FG_THREADS / ROWS;
+            const uint32_t f = first + (uint32_t)(stage * FG_BK + j * KSTEP) * inc;
+            const bool in = row_ok && k_begin + stage * FG_BK + kk0 + j * KSTEP < kend;
+            r[j >> 2][j & 3] = in ? sq5_unit(sq5_tail(f)) : 0.0f;
+        }
     }
-    __device__ __forceinline__ void store(float *__restrict__ tile) const
+    __device__ __forceinline__ void store(int stage, float *__restrict__ tile) const
     {
         const int t = threadIdx.x & (FG_THREADS - 1);
         if (SRC == FG_KCONT) {
 #pragma unroll
             for (int h = 0; h < NV; ++h) {
                 const int idx = h * FG_THREADS + t, row = idx >> 2, kq = idx & 3;
+                const Piece v = whole(stage, h);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) tile[(kq * 4 + j) * LD + row] = r[h][j];
+                for (int j = 0; j < 4; ++j) tile[(kq * 4 + j) * LD + row] = v[j];
             }
         } else if (SRC == FG_MCONT) {
 #pragma unroll
             for (int h = 0; h < NV; ++h) {
                 const int idx = h * FG_THREADS + t, kk = idx / (ROWS / 4), r4 = (idx % (ROWS / 4)) * 4;
-                *reinterpret_cast<f32x4 *>(tile + kk * LD + r4) = r[h];
+                *reinterpret_cast<Piece *>(tile + kk * LD + r4) = whole(stage, h);
             }
         } else {
             constexpr int KSTEP = FG_THREADS / ROWS;
@@ -255,53 +303,50 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
             for (int j = 0; j < NV * 4; ++j) tile[(kk0 + j * KSTEP) * LD + row] = r[j >> 2][j & 3];
         }
     }
-    // SPLIT: four of the thread's values into the planes, 8 bytes each, at element offset `at` of a plane.  Values that come from a
-    // bf16 matrix are their own first part and the other two are zero: only the first plane is written (and read, see the kernel).
-    __device__ __forceinline__ bool one_plane() const { return !HASHED && es == 2; }
-    template <bool ONE, bool FINITE> __device__ __forceinline__ void put4(bf16_t *__restrict__ tile, int at, const f32x4 &v) const
+    // SPLIT: four of the thread's values into the planes, 8 bytes each, at element offset `at` of a plane.
+    template <bool FINITE> __device__ __forceinline__ void put4(bf16_t *__restrict__ tile, int at, const Piece &v) const
     {
-        if (ONE) {
-            *reinterpret_cast<uint2 *>(tile + at) = make_uint2((__float_as_uint(v[1]) & 0xffff0000u) | (__float_as_uint(v[0]) >> 16),
-                                                               (__float_as_uint(v[3]) & 0xffff0000u) | (__float_as_uint(v[2]) >> 16));
-            return;
-        }
-        uint2 h, m, l;
-        if (FINITE) {
-            fg_split3(v[0], v[1], h.x, m.x, l.x);
-            fg_split3(v[2], v[3], h.y, m.y, l.y);
+        if constexpr (ONE) {
+            *reinterpret_cast<u32x2 *>(tile + at) = v;
         } else {
-            uint32_t p[4][3];
+            uint2 h, m, l;
+            if (FINITE) {
+                fg_split3(v[0], v[1], h.x, m.x, l.x);
+                fg_split3(v[2], v[3], h.y, m.y, l.y);
+            } else {
+                uint32_t p[4][3];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) fg_split3_any(v[j], p[j][0], p[j][1], p[j][2]);
-            h = make_uint2(p[1][0] | (p[0][0] >> 16), p[3][0] | (p[2][0] >> 16));
-            m = make_uint2(p[1][1] | (p[0][1] >> 16), p[3][1] | (p[2][1] >> 16));
-            l = make_uint2(p[1][2] | (p[0][2] >> 16), p[3][2] | (p[2][2] >> 16));
+                for (int j = 0; j < 4; ++j) fg_split3_any(v[j], p[j][0], p[j][1], p[j][2]);
+                h = make_uint2(p[1][0] | (p[0][0] >> 16), p[3][0] | (p[2][0] >> 16));
+                m = make_uint2(p[1][1] | (p[0][1] >> 16), p[3][1] | (p[2][1] >> 16));
+                l = make_uint2(p[1][2] | (p[0][2] >> 16), p[3][2] | (p[2][2] >> 16));
+            }
+            *reinterpret_cast<uint2 *>(tile + at) = h;
+            *reinterpret_cast<uint2 *>(tile + PLANE + at) = m;
+            *reinterpret_cast<uint2 *>(tile + 2 * PLANE + at) = l;
         }
-        *reinterpret_cast<uint2 *>(tile + at) = h;
-        *reinterpret_cast<uint2 *>(tile + PLANE + at) = m;
-        *reinterpret_cast<uint2 *>(tile + 2 * PLANE + at) = l;
     }
-    template <bool ONE, bool FINITE> __device__ __forceinline__ void store_split(bf16_t *__restrict__ tile) const
+    template <bool FINITE> __device__ __forceinline__ void store_split(int stage, bf16_t *__restrict__ tile) const
     {
         const int t = threadIdx.x & (FG_THREADS - 1);
         if (SRC == FG_KCONT) {
 #pragma unroll
             for (int h = 0; h < NV; ++h) {   // contraction values 4 kq .. 4 kq + 3 of a row
                 const int idx = h * FG_THREADS + t, row = idx >> 2, kq = idx & 3;
-                put4<ONE, FINITE>(tile, ((kq >> 1) * ROWS + row) * 8 + (kq & 1) * 4, r[h]);
+                put4<FINITE>(tile, ((kq >> 1) * ROWS + row) * 8 + (kq & 1) * 4, whole(stage, h));
             }
         } else if (SRC == FG_MCONT) {
 #pragma unroll
             for (int h = 0; h < NV; ++h) {   // four consecutive rows at one contraction value
                 const int idx = h * FG_THREADS + t, kk = idx / (ROWS / 4), r4 = (idx % (ROWS / 4)) * 4;
-                put4<ONE, FINITE>(tile, kk * LDM + r4, r[h]);
+                put4<FINITE>(tile, kk * LDM + r4, whole(stage, h));
             }
         } else {
             const int row = t % ROWS;
 #pragma unroll
             for (int h = 0; h < NV; ++h) {   // contraction values kk0 + 4 h .. + 3 of a row
                 const int kk = kk0 + 4 * h;
-                put4<ONE, FINITE>(tile, ((kk >> 3) * ROWS + row) * 8 + (kk & 7), r[h]);
+                put4<FINITE>(tile, ((kk >> 3) * ROWS + row) * 8 + (kk & 7), r[h]);
             }
         }
     }
@@ -333,11 +378,13 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false> struct FgOperand {
 // matters little.
 // Results leave with streaming stores: they would be written back from L2 at the end of the kernel otherwise, after the last
 // block (y of that layer, 25 MB: 26.4 -> 24.8 us).
-template <int BM, int G, int ASRC, int BSRC, int EPI, bool VEC, bool SPLIT = false, bool ANY16 = false>
+// AES, BES: bytes per element of the two matrices (SPLIT: 4, or 2, bf16; otherwise 0, see FgOperand).
+template <int BM, int G, int ASRC, int BSRC, int EPI, bool VEC, bool SPLIT, int AES, int BES>
 __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kernel(FgParams p)
 {
-    typedef FgOperand<BM, ASRC, VEC, SPLIT> PA;
-    typedef FgOperand<FG_BN, BSRC, VEC, SPLIT> PB;
+    typedef FgOperand<BM, ASRC, VEC, SPLIT, AES> PA;
+    typedef FgOperand<FG_BN, BSRC, VEC, SPLIT, BES> PB;
+    constexpr bool ANY16 = PA::ONE || PB::ONE;
     constexpr int MI = BM / 64, NI = 2, STAGE = (PA::TILE_BYTES + PB::TILE_BYTES) / 4;   // floats
     static_assert(G == 1 || SPLIT, "groups: the bf16 matrix instructions only");
     constexpr int UNITS = MI * NI * 2;   // a wave's accumulators in units of 8 registers: what the groups share out at the end
@@ -353,8 +400,8 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
     const int k_begin = k_first + group * nstage * FG_BK, kend = min(k_last, k_begin + nstage * FG_BK);
     PA pa;
     PB pb;
-    pa.init(p.a, p.lda, p.a_bytes, m0, p.M, k_begin, kend, p.seed, p.nsR, p.nsK, p.a_es);
-    pb.init(p.b, p.ldb, p.b_bytes, n0, p.N, k_begin, kend, p.seed, p.nsR, p.nsK, p.b_es);
+    pa.init(p.a, p.lda, p.a_bytes, m0, p.M, p.K, k_begin, kend, nstage, p.seed, p.nsR, p.nsK, p.a_es);
+    pb.init(p.b, p.ldb, p.b_bytes, n0, p.N, p.K, k_begin, kend, nstage, p.seed, p.nsR, p.nsK, p.b_es);
     // The five smaller products of the parts in sums of their own (low), where registers allow it: the large sum is then rounded once a
     // stage and not six times.  Distance from 64 bits, 13 layers of 32 to 1024 tokens with k <= 64, input gradient: 0.60 times that of
     // fp32 multiplications and additions one after the other, as the vector-ALU kernels do them (1.01 times with one sum, 1.15 with
@@ -363,20 +410,19 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
     constexpr bool APART = SPLIT && BM == 64 && G > 1 && !ANY16;
     f32x16 acc[MI][NI], low[MI][NI];
     if (threadIdx.x == 0) not_finite = 0;   // seen by everybody behind the first stage's barrier
-    // The stage loop, once per number of planes of the two sides (known per launch, not per kernel: a side that comes from a
-    // bf16 matrix has one plane), so that each copy is straight-line code between its barriers.
-    // ... and, for fp32 matrices, once more for sums that are not finite (fg_split3).
-    auto stages = [&](auto a_one, auto b_one, auto finite) __attribute__((always_inline)) {
-        constexpr int AP = decltype(a_one)::value ? 1 : 3, BP = decltype(b_one)::value ? 1 : 3;
+    // The stage loop; for fp32 matrices once more for sums that are not finite (fg_split3).  A side that comes from a bf16 matrix has one
+    // plane.
+    auto stages = [&](auto finite) __attribute__((always_inline)) {
+        constexpr int AP = PA::ONE ? 1 : 3, BP = PB::ONE ? 1 : 3;
         constexpr bool FINITE = decltype(finite)::value;
         for (int s = 0; s < nstage; ++s) {
             float *As = lds + (s & 1) * STAGE, *Bs = As + PA::TILE_BYTES / 4;
             if (SPLIT) {
-                pa.template store_split<AP == 1, PA::HASHED || FINITE>(reinterpret_cast<bf16_t *>(As));
-                pb.template store_split<BP == 1, PB::HASHED || FINITE>(reinterpret_cast<bf16_t *>(Bs));
+                pa.template store_split<PA::HASHED || FINITE>(s, reinterpret_cast<bf16_t *>(As));
+                pb.template store_split<PB::HASHED || FINITE>(s, reinterpret_cast<bf16_t *>(Bs));
             } else {
-                pa.store(As);
-                pb.store(Bs);
+                pa.store(s, As);
+                pb.store(s, Bs);
             }
             __syncthreads();   // also: every wave is done reading the other buffer (the stage before this one)
             const bool more = s + 1 < nstage;
@@ -454,8 +500,6 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
             }
         }
     };
-    typedef std::integral_constant<bool, true> One;
-    typedef std::integral_constant<bool, false> Three;
     auto product = [&](auto finite) __attribute__((always_inline)) {
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi)
@@ -465,18 +509,7 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
                 for (int e = 0; e < 16; ++e) acc[mi][ni][e] = low[mi][ni][e] = 0.0f;
         pa.load(0);
         pb.load(0);
-        if (!SPLIT || !ANY16) {   // ANY16: one of the matrices is bf16 (only then is the choice compiled in)
-            stages(Three{}, Three{}, finite);
-        } else {
-            const bool a1 = pa.one_plane(), b1 = pb.one_plane();
-            if (PA::HASHED || !a1) {
-                if (PB::HASHED || !b1) stages(Three{}, Three{}, finite);
-                else stages(Three{}, One{}, finite);
-            } else {
-                if (PB::HASHED || !b1) stages(One{}, Three{}, finite);
-                else stages(One{}, One{}, finite);
-            }
-        }
+        stages(finite);
         if (APART) {
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi)
@@ -673,24 +706,37 @@ struct FgProduct {
 #define FG_LAUNCH_GROUPS(BM_, G_, EPI_)                                                                               \
     do {                                                                                                            \
         const int nt = FG_THREADS * G_;                                                                             \
-        if (any16) {                                                                                                \
-            if (vec) f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, true, true, true><<<grid, nt, 0, s>>>(p);           \
-            else f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, false, true, true><<<grid, nt, 0, s>>>(p);              \
+        auto of = [&](auto aes_, auto bes_) {                                                                       \
+            constexpr int AES = decltype(aes_)::value, BES = decltype(bes_)::value;                                 \
+            if (vec) f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, true, true, AES, BES><<<grid, nt, 0, s>>>(p);       \
+            else f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, false, true, AES, BES><<<grid, nt, 0, s>>>(p);          \
+        };                                                                                                          \
+        typedef std::integral_constant<int, 4> Wide;                                                                \
+        typedef std::integral_constant<int, 2> Narrow;                                                              \
+        if (a16) {                                                                                                  \
+            if constexpr (Groups::a16_b16) { if (b16) { of(Narrow{}, Narrow{}); break; } }                          \
+            if constexpr (Groups::a16_b32) of(Narrow{}, Wide{});                                                    \
+        } else if (b16) {                                                                                           \
+            if constexpr (Groups::a32_b16) of(Wide{}, Narrow{});                                                    \
         } else {                                                                                                    \
-            if (vec) f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, true, true><<<grid, nt, 0, s>>>(p);                 \
-            else f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, false, true><<<grid, nt, 0, s>>>(p);                    \
+            of(Wide{}, Wide{});                                                                                     \
         }                                                                                                           \
     } while (0)
 #define FG_LAUNCH(BM_, EPI_)                                                                                        \
     do {                                                                                                            \
         if (q.split) FG_LAUNCH_GROUPS(BM_, 1, EPI_);                                                                \
-        else if (vec) f32_gemm_kernel<BM_, 1, ASRC, BSRC, EPI_, true><<<grid, FG_THREADS, 0, s>>>(p);               \
-        else f32_gemm_kernel<BM_, 1, ASRC, BSRC, EPI_, false><<<grid, FG_THREADS, 0, s>>>(p);                       \
+        else if (vec) f32_gemm_kernel<BM_, 1, ASRC, BSRC, EPI_, true, false, 0, 0><<<grid, FG_THREADS, 0, s>>>(p);  \
+        else f32_gemm_kernel<BM_, 1, ASRC, BSRC, EPI_, false, false, 0, 0><<<grid, FG_THREADS, 0, s>>>(p);          \
     } while (0)
 // What is built for a pair of sources: four groups per block (their buffers do not fit in LDS where a side is read
 // across its rows: its planes are padded), and the epilogues that add a bias and a random-bias share.
 template <int ASRC, int BSRC> struct FgGroups {
     static constexpr bool four = ASRC != FG_MCONT && BSRC != FG_MCONT;
+    // which sides may be bf16 matrices: x and dy are as the coefficients are, z and t are fp32
+    static constexpr bool matrices = ASRC != FG_NOISE_I && (BSRC == FG_KCONT || BSRC == FG_MCONT);
+    static constexpr bool a16_b16 = matrices && BSRC == FG_MCONT;                               // t = dy . C, dW = dy^T . x
+    static constexpr bool a16_b32 = ASRC == FG_MCONT || (ASRC == FG_KCONT && !matrices);        // dC = dy^T . z, z = x . N^T, W = C . N
+    static constexpr bool a32_b16 = BSRC == FG_KCONT;                                           // y = z . C^T, W^T = N^T . C^T
     static constexpr bool biased = ASRC == FG_KCONT && BSRC == FG_KCONT, scaled = ASRC == FG_NOISE_I || BSRC == FG_NOISE_I;
 };
 template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_t s, const char *name)
@@ -736,7 +782,8 @@ template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_
         return fg_aligned16(m) && ld % 4 == 0 && (src == FG_KCONT ? q.K % 4 == 0 : rows % 4 == 0);
     };
     const bool vec = vec_ok(ASRC, q.a, q.lda, q.M) && vec_ok(BSRC, q.b, q.ldb, q.N);   // bf16 matrices: 8-byte pieces of four values
-    const bool any16 = q.a_es == 2 || ((BSRC == FG_KCONT || BSRC == FG_MCONT) && q.b_es == 2);   // the A side is always a matrix
+    const bool a16 = (ASRC == FG_KCONT || ASRC == FG_MCONT) && q.a_es == 2, b16 = (BSRC == FG_KCONT || BSRC == FG_MCONT) && q.b_es == 2;
+    if (q.split && ((a16 && b16) ? !Groups::a16_b16 : a16 ? !Groups::a16_b32 : b16 && !Groups::a32_b16)) return RDB_E_UNSUPPORTED;
     if (cdiv(q.N, FG_BN) > 65535) return RDB_E_UNSUPPORTED;   // the grid's y
     const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)splits);
     auto run = [&](auto epi_) {

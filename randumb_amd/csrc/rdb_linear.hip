@@ -467,7 +467,7 @@ static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d)
     if (d->act_dtype == RDB_BF16 && d->coef_rows != 0 && (d->in_f % 8 || d->out_f % 8 || d->k % 8) &&
         (op == RDB_OP_LINEAR_FWD || op == RDB_OP_LINEAR_BWD_DX || op == RDB_OP_LINEAR_BWD_DCOEF)) {
         // bf16 layers the bf16 factored kernels do not take (sizes that are not multiples of 8): the fp32 matrix-core kernels
-        // with bf16 matrices read value by value
+        // with bf16 matrices read at any address
         rdb_linear_desc dd = *d;
         if (op == RDB_OP_LINEAR_BWD_DCOEF) dd.coef_dtype = RDB_BF16;
         return linear_f32_workspace(op, &dd, num_compute_units());
@@ -655,7 +655,7 @@ extern "C" int rdb_linear_bwd_dx(void *dx, int64_t lddx, const void *dy, int64_t
         df.algo = RDB_ALGO_FACTORED;
         rc = linear_dx_factored(dx, lddx, dy, lddy, coef, scale_bias, &df, num_compute_units(), workspace, workspace_bytes, (hipStream_t)stream);
         if (rc != RDB_E_UNSUPPORTED) return rc;
-        if (d->act_dtype == RDB_BF16) {   // sizes that are not multiples of 8: the fp32 matrix cores, reading bf16 value by value
+        if (d->act_dtype == RDB_BF16) {   // sizes that are not multiples of 8: the fp32-accurate products, reading bf16 at any address
             rc = linear_dx_f32(dx, lddx, dy, lddy, coef, scale_bias, d, num_compute_units(), workspace, workspace_bytes, (hipStream_t)stream);
             if (rc != RDB_E_UNSUPPORTED) return rc;
         }
@@ -838,7 +838,7 @@ extern "C" int rdb_linear_bwd_dcoef(float *dcoef, float *d_scale_bias, const voi
         if (rc != RDB_E_UNSUPPORTED) return rc;
     }
     if (d->algo == RDB_ALGO_AUTO && d->act_dtype == RDB_BF16) {
-        // sizes that are not multiples of 8: the fp32 matrix cores, reading bf16 value by value (they overwrite what was cleared)
+        // sizes that are not multiples of 8: the fp32-accurate products, reading bf16 at any address (they overwrite what was cleared)
         rc = linear_dcoef_f32(dcoef, d_scale_bias, dy, lddy, x, ldx, d, num_compute_units(), workspace, workspace_bytes, s);
         if (rc != RDB_E_UNSUPPORTED) return rc;
     }

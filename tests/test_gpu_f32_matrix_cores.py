@@ -136,6 +136,33 @@ def test_unaligned_views(hip, oracle):
     assert rel_l2(dc.cpu().numpy(), want_dc) < F32_TOL
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("in_f,out_f,k", [(1, 2, 3), (2, 9, 1), (3, 5, 2), (4, 6, 5), (5, 3, 7), (17, 15, 18), (66, 131, 19), (129, 65, 33), (259, 126, 65)])
+def test_rows_that_end_inside_a_piece_of_four(hip, oracle, in_f, out_f, k, dtype):
+    """Extents of which 1, 2, 3 or all 4 values of a row's last piece exist, and rows of fewer than four values, with NaNs behind every row.
+    Every product accumulates in fp32 (1e-5); what is stored as bf16 is rounded once (2^-9)."""
+    from randumb_amd._lib import RDB_ALGO_AUTO, RDB_ALGO_FACTORED
+
+    algo = RDB_ALGO_FACTORED if dtype == torch.float32 else RDB_ALGO_AUTO   # the factored form of bf16 is that of whole multiples of 8
+    T, seed = 131, 23
+    x, dy, coef, _ = (v.to(dtype) for v in _inputs(T, in_f, out_f, k, seed))
+    def behind_nans(v):
+        wide = torch.full((v.shape[0], v.shape[1] + 3), float("nan"), device="cuda", dtype=dtype)
+        wide[:, :v.shape[1]] = v.cuda()
+        return wide[:, :v.shape[1]]
+    xs, dys, cc = behind_nans(x), behind_nans(dy), coef.cuda()
+    want_y = oracle.linear_fwd(x.float().numpy(), coef.float().numpy(), in_f, out_f, seed)
+    want_dx, want_dc, _ = oracle.linear_bwd(x.float().numpy(), dy.float().numpy(), coef.float().numpy(), in_f, out_f, seed)
+    tol = F32_TOL if dtype == torch.float32 else 2.0**-9
+    print(f"case f32 matrix cores edges in={in_f} out={out_f} k={k} {dtype}", flush=True)
+    y = hip.linear_fwd(xs, cc, in_f, out_f, in_f, 1, seed, algo=algo)
+    assert rel_l2(y.float().cpu().numpy(), want_y) < tol
+    dx = hip.linear_bwd_dx(dys, cc, in_f, out_f, in_f, 1, seed, algo=algo)
+    assert rel_l2(dx.float().cpu().numpy(), want_dx) < tol
+    dc, _ = hip.linear_bwd_dcoef(dys, xs, k, out_f, in_f, out_f, in_f, 1, seed, algo=algo)
+    assert rel_l2(dc.cpu().numpy(), want_dc) < F32_TOL
+
+
 def test_layer_level_fp32(hip, oracle):
     """SillyLinear(matrix_coef=True) in fp32 at a GPT-like slice: forward, input gradient and coefficient gradient through autograd."""
     from randumb_amd.SillyLayers import SillyLinear

@@ -56,21 +56,41 @@ template <typename V> __device__ __forceinline__ V sum_in_order(const float *__r
 }
 
 // out[i] = part[0][i] + part[1][i] + ... in split order, four values per thread (n4 groups of four, then the n % 4 last values
-// one thread each); out fp32, or bf16 (rounded once)
-__global__ __launch_bounds__(256) void f32_sum_splits_kernel(void *__restrict__ out, int out_bf16, const float *__restrict__ part, int64_t n, int64_t stride,
-                                                             int splits, int vec)
+// one thread each); out fp32, or bf16 (rounded once).  One or two such sums a launch: the second one's blocks follow.
+struct FgSum {
+    void *out;
+    const float *part;
+    int64_t n, stride;   // values, floats between the partial matrices
+    int out_bf16, splits, vec;
+    int blocks;          // 0: no such sum
+};
+__global__ __launch_bounds__(256) void f32_sum_splits_kernel(FgSum a, FgSum b)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, n4 = vec ? n / 4 : 0;
+    const bool second = (int)blockIdx.x >= a.blocks;
+    const FgSum &q = second ? b : a;
+    const int64_t i = (int64_t)((int)blockIdx.x - (second ? a.blocks : 0)) * 256 + threadIdx.x, n4 = q.vec ? q.n / 4 : 0;
     if (i < n4) {
-        const f32x4 v = sum_in_order<f32x4>(part + i * 4, stride, splits);
-        if (out_bf16) store4<bf16_t>(static_cast<bf16_t *>(out) + i * 4, v[0], v[1], v[2], v[3]);
-        else *reinterpret_cast<f32x4 *>(static_cast<float *>(out) + i * 4) = v;
-    } else if (n4 * 4 + (i - n4) < n) {
+        const f32x4 v = sum_in_order<f32x4>(q.part + i * 4, q.stride, q.splits);
+        if (q.out_bf16) store4<bf16_t>(static_cast<bf16_t *>(q.out) + i * 4, v[0], v[1], v[2], v[3]);
+        else *reinterpret_cast<f32x4 *>(static_cast<float *>(q.out) + i * 4) = v;
+    } else if (n4 * 4 + (i - n4) < q.n) {
         const int64_t e = n4 * 4 + (i - n4);
-        const float v = sum_in_order<float>(part + e, stride, splits);
-        if (out_bf16) static_cast<bf16_t *>(out)[e] = f32_to_bf16(v);
-        else static_cast<float *>(out)[e] = v;
+        const float v = sum_in_order<float>(q.part + e, q.stride, q.splits);
+        if (q.out_bf16) static_cast<bf16_t *>(q.out)[e] = f32_to_bf16(v);
+        else static_cast<float *>(q.out)[e] = v;
     }
+}
+static FgSum fg_sum(void *out, int out_bf16, const float *part, int64_t n, int64_t stride, int splits)
+{
+    if (splits <= 1) return {};
+    const int vec = fg_aligned16(out) ? 1 : 0;   // the partial matrices are 256-byte aligned
+    return {out, part, n, stride, out_bf16, splits, vec, (int)cdiv(vec ? n / 4 + n % 4 : n, 256)};
+}
+static int fg_launch_sums(const FgSum &a, const FgSum &b, hipStream_t s)
+{
+    if (!(a.blocks + b.blocks)) return RDB_OK;
+    f32_sum_splits_kernel<<<(unsigned)(a.blocks + b.blocks), 256, 0, s>>>(a, b);
+    return check_launch("f32_sum_splits_kernel");
 }
 
 // 1 (default): the linear layers' products run as six bf16 matrix instructions on three-way splits of their operands
@@ -140,9 +160,34 @@ template <int ASRC, int BSRC> static int fg_launch_ranges(FgProduct q, int room,
     q.kchunk = cdiv(cdiv(q.K, plan.ranges), FG_BK) * FG_BK;   // every range holds something (fg_plan)
     q.split_stride = stride;
     if (int rc = fg_launch<ASRC, BSRC>(q, num_cus, s, name)) return rc;
-    const int vec = fg_aligned16(out) ? 1 : 0;   // the partial matrices are 256-byte aligned
-    f32_sum_splits_kernel<<<(unsigned)cdiv(vec ? n / 4 + n % 4 : n, 256), 256, 0, s>>>(out, out_bf16, part, n, stride, plan.ranges, vec);
-    return check_launch("f32_sum_splits_kernel");
+    return fg_launch_sums(fg_sum(out, out_bf16, part, n, stride, plan.ranges), FgSum{}, s);
+}
+
+// Two such products that do not need each other, in one launch, and their sums in one: t = dy . C and dC = dy^T . z.
+int fg_launch_pair(const FgProduct &t, const FgProduct &dc, hipStream_t s);   // rdb_f32_pair.hip
+static int fg_launch_pair_ranges(FgProduct t, int t_room, float *t_part, int64_t t_stride, FgProduct dc, int dc_room, float *dc_part, int64_t dc_stride,
+                                 int num_cus, hipStream_t s)
+{
+    const FgPairPlan plan = fg_plan_pair({t.M, dc.M}, {t.N, dc.N}, {t.K, dc.K}, num_cus, {t_room, dc_room}, t.a_es == 2);
+    FgProduct *const q[2] = {&t, &dc};
+    float *const part[2] = {t_part, dc_part};
+    const int64_t stride[2] = {t_stride, dc_stride};
+    FgSum sum[2];
+    for (int i = 0; i < 2; ++i) {
+        FgProduct &p = *q[i];
+        const int r = plan.ranges[i];
+        p.bm = plan.bm;
+        p.groups = plan.groups;
+        p.kchunk = fg_chunk(p.K, r);
+        sum[i] = fg_sum(p.out, p.out_bf16, part[i], p.M * p.N, stride[i], r);
+        if (r > 1) {
+            p.out = part[i];
+            p.out_bf16 = 0;
+            p.split_stride = stride[i];
+        }
+    }
+    if (int rc = fg_launch_pair(t, dc, s)) return rc;
+    return fg_launch_sums(sum[0], sum[1], s);
 }
 
 // z[T x k] = src[T x in_f] . N^T; the partial matrices of its ranges go to `part` (room for max_ranges of them, up256(T k 4)
@@ -181,25 +226,65 @@ int linear_fwd_f32(void *y, int64_t ldy, const void *x, int64_t ldx, const void 
     return fg_launch<FG_KCONT, FG_NOISE_1D>(qr, num_cus, s, "f32_gemm_kernel (y += s x . R^T)");
 }
 
+// t[T x k] = dy[T x out_f] . C: the B side's rows are coefficients, read across the rows of C
+static FgProduct fg_t(float *t, const void *dy, int64_t lddy, const void *coef, const rdb_linear_desc *d)
+{
+    FgProduct q = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, (const float *)coef, d->k, d->out_f * d->k, t, d->k, nullptr,
+                   d->tokens, d->k, d->out_f, 0, 0, 0, 0, d->seed};
+    q.a_es = fg_es(d->act_dtype);
+    q.b_es = fg_es(d->coef_dtype);
+    return q;
+}
+// dx[T x in_f] = t . N: the B side's rows are input features, hashed
+static int fg_dx_from_t(void *dx, int64_t lddx, const float *t, const rdb_linear_desc *d, int num_cus, hipStream_t s)
+{
+    FgProduct q = {t, d->k, d->tokens * d->k, nullptr, 0, 0, (float *)dx, lddx, nullptr, d->tokens, d->in_f, d->k, 0, 0, 0, 0, d->seed};
+    q.out_bf16 = d->act_dtype == RDB_BF16;
+    return fg_launch<FG_KCONT, FG_NOISE_I>(q, num_cus, s, "f32_gemm_kernel (dx = t . N)");
+}
+// dC[out_f x k] = dy^T . z: both sides are read across their rows (the contraction runs over the tokens)
+static FgProduct fg_dc(void *dcoef, int dcoef_dtype, const void *dy, int64_t lddy, const float *z, const rdb_linear_desc *d)
+{
+    FgProduct q = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, z, d->k, d->tokens * d->k, (float *)dcoef, d->k, nullptr,
+                   d->out_f, d->k, d->tokens, 0, 0, 0, 0, d->seed};
+    q.a_es = fg_es(d->act_dtype);
+    q.out_bf16 = dcoef_dtype == RDB_BF16;
+    return q;
+}
+int linear_dx_f32(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *coef, const void *scale_bias, const rdb_linear_desc *d,
+                  int num_cus, void *workspace, int64_t workspace_bytes, hipStream_t s);
+// dx and / or dC (each NULL where it is not wanted) from dy, z and C; dc_part: room for dC's partial matrices
+static int fg_backward(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, const void *dy, int64_t lddy, const float *z, const void *coef,
+                       const rdb_linear_desc *d, int num_cus, void *workspace, int64_t workspace_bytes, float *dc_part, hipStream_t s)
+{
+    const int room = dc_room(d, num_cus);
+    const int64_t dc_stride = up256(d->out_f * d->k * 4) / 4;
+    if (dx && dcoef && f32_split_mode()) {
+        float *t = (float *)workspace;
+        const int64_t zt = up256(d->tokens * d->k * 4) / 4;
+        if (int rc = fg_launch_pair_ranges(fg_t(t, dy, lddy, coef, d), zt_room(d, d->out_f, num_cus), t + zt, zt, fg_dc(dcoef, dcoef_dtype, dy, lddy, z, d),
+                                           room, dc_part, dc_stride, num_cus, s))
+            return rc;
+        return fg_dx_from_t(dx, lddx, t, d, num_cus, s);
+    }
+    if (dx) {
+        if (int rc = linear_dx_f32(dx, lddx, dy, lddy, coef, nullptr, d, num_cus, workspace, workspace_bytes, s)) return rc;
+    }
+    if (!dcoef) return RDB_OK;
+    return fg_launch_ranges<FG_MCONT, FG_MCONT>(fg_dc(dcoef, dcoef_dtype, dy, lddy, z, d), room, dc_part, dc_stride, num_cus, s, "f32_gemm_kernel (dC = dy^T . z)");
+}
+
 int linear_dx_f32(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *coef, const void *scale_bias, const rdb_linear_desc *d,
                   int num_cus, void *workspace, int64_t workspace_bytes, hipStream_t s)
 {
     if (!fg_ok(d) || !fg_wanted(d) || !fg_ws_ok(RDB_OP_LINEAR_BWD_DX, d, num_cus, workspace, workspace_bytes)) return RDB_E_UNSUPPORTED;
     if (d->tokens * lddx >= (1ll << 29) || d->tokens * lddy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     float *t = (float *)workspace;
-    // t[T x k] = dy[T x out_f] . C: the B side's rows are coefficients, read across the rows of C
-    FgProduct q1 = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, (const float *)coef, d->k, d->out_f * d->k, t, d->k, nullptr,
-                    d->tokens, d->k, d->out_f, 0, 0, 0, 0, d->seed};
     const int b16 = d->act_dtype == RDB_BF16;
-    q1.a_es = fg_es(d->act_dtype);
-    q1.b_es = fg_es(d->coef_dtype);
     const int64_t zt = up256(d->tokens * d->k * 4) / 4;
-    if (int rc = fg_launch_ranges<FG_KCONT, FG_MCONT>(q1, zt_room(d, d->out_f, num_cus), t + zt, zt, num_cus, s, "f32_gemm_kernel (t = dy . C)")) return rc;
-    // dx[T x in_f] = t . N: the B side's rows are input features, hashed
-    FgProduct q2 = {t, d->k, d->tokens * d->k, nullptr, 0, 0, (float *)dx, lddx, nullptr, d->tokens, d->in_f, d->k,
-                    0, 0, 0, 0, d->seed};
-    q2.out_bf16 = b16;
-    if (int rc = fg_launch<FG_KCONT, FG_NOISE_I>(q2, num_cus, s, "f32_gemm_kernel (dx = t . N)")) return rc;
+    if (int rc = fg_launch_ranges<FG_KCONT, FG_MCONT>(fg_t(t, dy, lddy, coef, d), zt_room(d, d->out_f, num_cus), t + zt, zt, num_cus, s, "f32_gemm_kernel (t = dy . C)"))
+        return rc;
+    if (int rc = fg_dx_from_t(dx, lddx, t, d, num_cus, s)) return rc;
     if (!scale_bias) return RDB_OK;
     // dx += s * dy . R: the B side's rows are input features, index o * in_f + i
     FgProduct qr = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, nullptr, 0, 0, (float *)dx, lddx, nullptr, d->tokens, d->in_f, d->out_f,
@@ -222,14 +307,10 @@ int linear_dcoef_f32(float *dcoef, float *d_scale_bias, const void *dy, int64_t 
     if (d->tokens * ldx >= (1ll << 29) || d->tokens * lddy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     float *z = (float *)workspace;
     if (int rc = fg_project(z, (const float *)x, ldx, &dd, num_cus, s)) return rc;
-    // dC[out_f x k] = dy^T . z: both sides are read across their rows (the contraction runs over the tokens)
     const int zs = zt_room(&dd, d->in_f, num_cus);
     float *part = reinterpret_cast<float *>(static_cast<char *>(workspace) + up256(d->tokens * d->k * 4) * (zs > 1 ? 1 + zs : 1));
-    FgProduct q = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, z, d->k, d->tokens * d->k, dcoef, d->k, nullptr,
-                   d->out_f, d->k, d->tokens, 0, 0, 0, 0, d->seed};
     const int dcr = dc_room(&dd, num_cus);
-    q.a_es = fg_es(d->act_dtype);
-    if (int rc = fg_launch_ranges<FG_MCONT, FG_MCONT>(q, dcr, part, up256(d->out_f * d->k * 4) / 4, num_cus, s, "f32_gemm_kernel (dC = dy^T . z)")) return rc;
+    if (int rc = fg_launch_ranges<FG_MCONT, FG_MCONT>(fg_dc(dcoef, RDB_F32, dy, lddy, z, &dd), dcr, part, up256(d->out_f * d->k * 4) / 4, num_cus, s, "f32_gemm_kernel (dC = dy^T . z)")) return rc;
     if (!d_scale_bias) return RDB_OK;
     // <dy, x . R^T>: the random-bias product once more, each block reducing its tile against dy's; then the blocks in order
     float *dots = part + (dcr > 1 ? (int64_t)dcr * (up256(d->out_f * d->k * 4) / 4) : 0);
@@ -335,18 +416,9 @@ int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, fl
     char *const dc_part = static_cast<char *>(workspace) + linear_f32_workspace(RDB_OP_LINEAR_BWD_DX, d, num_cus);
     const int r = dc_room(d, num_cus);
     float *const dots = reinterpret_cast<float *>(dc_part + (r > 1 ? (int64_t)r * up256(d->out_f * d->k * 4) : 0));
-    if (dx) {
-        if (int rc = linear_dx_f32(dx, lddx, dy, lddy, coef, nullptr, d, num_cus, workspace, workspace_bytes, s)) return rc;
-    }
-    if (dcoef) {
-        FgProduct q = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, static_cast<const float *>(kept), d->k, d->tokens * d->k, (float *)dcoef, d->k,
-                       nullptr, d->out_f, d->k, d->tokens, 0, 0, 0, 0, d->seed};
-        q.a_es = fg_es(d->act_dtype);
-        q.out_bf16 = dcoef_dtype == RDB_BF16;
-        if (int rc = fg_launch_ranges<FG_MCONT, FG_MCONT>(q, r, reinterpret_cast<float *>(dc_part), up256(d->out_f * d->k * 4) / 4, num_cus, s,
-                                                          "f32_gemm_kernel (dC = dy^T . z)"))
-            return rc;
-    }
+    if (int rc = fg_backward(dx, lddx, dcoef, dcoef_dtype, dy, lddy, static_cast<const float *>(kept), coef, d, num_cus, workspace, workspace_bytes,
+                             reinterpret_cast<float *>(dc_part), s))
+        return rc;
     if (!scale_bias || (!dx && !d_scale_bias)) return RDB_OK;
     FgProduct q;
     if (dx) {   // dx += s * dy . R, and <dy . R, x> on the way
@@ -451,14 +523,8 @@ int linear_bwd_projected_f32(void *dx, int64_t lddx, float *dcoef, const void *d
     if (!fg_state_ok(d) || !workspace || !fg_aligned16(workspace) || workspace_bytes < linear_f32_bwd_projected_workspace(d, num_cus))
         return RDB_E_UNSUPPORTED;
     if (d->tokens * lddy >= (1ll << 29) || (dx && d->tokens * lddx >= (1ll << 29))) return RDB_E_UNSUPPORTED;
-    if (dx) {
-        if (int rc = linear_dx_f32(dx, lddx, dy, lddy, coef, nullptr, d, num_cus, workspace, workspace_bytes, s)) return rc;
-    }
     float *part = reinterpret_cast<float *>(static_cast<char *>(workspace) + linear_f32_workspace(RDB_OP_LINEAR_BWD_DX, d, num_cus));
-    FgProduct q = {(const float *)dy, lddy, (d->tokens - 1) * lddy + d->out_f, fg_state_z(state), d->k, d->tokens * d->k, dcoef, d->k, nullptr,
-                   d->out_f, d->k, d->tokens, 0, 0, 0, 0, d->seed};
-    return fg_launch_ranges<FG_MCONT, FG_MCONT>(q, dc_room(d, num_cus), part, up256(d->out_f * d->k * 4) / 4, num_cus, s,
-                                                "f32_gemm_kernel (dC = dy^T . z)");
+    return fg_backward(dx, lddx, dcoef, RDB_F32, dy, lddy, fg_state_z(state), coef, d, num_cus, workspace, workspace_bytes, part, s);
 }
 
 // ----------------------------------------------------------------------------------------------- materialise on the matrix cores

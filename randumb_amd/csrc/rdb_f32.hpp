@@ -379,23 +379,30 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false, int ES = 4> struct Fg
 // Results leave with streaming stores: they would be written back from L2 at the end of the kernel otherwise, after the last
 // block (y of that layer, 25 MB: 26.4 -> 24.8 us).
 // AES, BES: bytes per element of the two matrices (SPLIT: 4, or 2, bf16; otherwise 0, see FgOperand).
-template <int BM, int G, int ASRC, int BSRC, int EPI, bool VEC, bool SPLIT, int AES, int BES>
-__global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kernel(FgParams p)
-{
+// f32_gemm_block: what block (bx, by, bz) of a product does (gx: how many there are along x).  `lds`: FgBlock::LDS floats; not_finite: a
+// word of LDS.
+template <int BM, int G, int ASRC, int BSRC, bool VEC, bool SPLIT, int AES, int BES> struct FgBlock {
     typedef FgOperand<BM, ASRC, VEC, SPLIT, AES> PA;
     typedef FgOperand<FG_BN, BSRC, VEC, SPLIT, BES> PB;
-    constexpr bool ANY16 = PA::ONE || PB::ONE;
-    constexpr int MI = BM / 64, NI = 2, STAGE = (PA::TILE_BYTES + PB::TILE_BYTES) / 4;   // floats
+    static constexpr int MI = BM / 64, NI = 2, STAGE = (PA::TILE_BYTES + PB::TILE_BYTES) / 4;   // floats
+    static constexpr int UNITS = MI * NI * 2;   // a wave's accumulators in units of 8 registers: what the groups share out at the end
+    static constexpr int EXCHANGE = (G - 1) * UNITS * 4 * 512;
+    static constexpr int LDS = 2 * STAGE * G > EXCHANGE ? 2 * STAGE * G : EXCHANGE;
     static_assert(G == 1 || SPLIT, "groups: the bf16 matrix instructions only");
-    constexpr int UNITS = MI * NI * 2;   // a wave's accumulators in units of 8 registers: what the groups share out at the end
-    constexpr int EXCHANGE = (G - 1) * UNITS * 4 * 512;
-    __shared__ __align__(16) float lds_all[2 * STAGE * G > EXCHANGE ? 2 * STAGE * G : EXCHANGE];
-    __shared__ int not_finite;   // some thread's sum is an infinity or a NaN
+};
+template <int BM, int G, int ASRC, int BSRC, int EPI, bool VEC, bool SPLIT, int AES, int BES>
+__device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, const int by, const int bz, const int gx, float *__restrict__ lds_all, int &not_finite)
+{
+    typedef FgBlock<BM, G, ASRC, BSRC, VEC, SPLIT, AES, BES> Block;
+    typedef typename Block::PA PA;
+    typedef typename Block::PB PB;
+    constexpr bool ANY16 = PA::ONE || PB::ONE;
+    constexpr int MI = Block::MI, NI = Block::NI, STAGE = Block::STAGE, UNITS = Block::UNITS;
     const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / FG_THREADS);
     float *lds = lds_all + group * 2 * STAGE;
     const int t = threadIdx.x & (FG_THREADS - 1), wave = t >> 6, lane = t & 63, r = lane & 31, g = lane >> 5, wm = wave >> 1, wn = wave & 1;
-    const int m0 = blockIdx.x * BM, n0 = blockIdx.y * FG_BN;   // the long extent (tokens, as a rule) on the grid's x
-    const int k_first = blockIdx.z * p.kchunk, k_last = min(p.K, k_first + p.kchunk);
+    const int m0 = bx * BM, n0 = by * FG_BN;   // the long extent (tokens, as a rule) on the grid's x
+    const int k_first = bz * p.kchunk, k_last = min(p.K, k_first + p.kchunk);
     const int nstage = ((k_last - k_first + FG_BK - 1) / FG_BK + G - 1) / G;   // of every group: the last one's may be empty
     const int k_begin = k_first + group * nstage * FG_BK, kend = min(k_last, k_begin + nstage * FG_BK);
     PA pa;
@@ -409,7 +416,7 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
     // quarter of their waves (2048 tokens x 768 -> 3072, k = 256: step 106.5 us against 104.4); their contractions are short.
     constexpr bool APART = SPLIT && BM == 64 && G > 1 && !ANY16;
     f32x16 acc[MI][NI], low[MI][NI];
-    if (threadIdx.x == 0) not_finite = 0;   // seen by everybody behind the first stage's barrier
+    if (SPLIT && !ANY16 && threadIdx.x == 0) not_finite = 0;   // seen by everybody behind the first stage's barrier
     // The stage loop; for fp32 matrices once more for sums that are not finite (fg_split3).  A side that comes from a bf16 matrix has one
     // plane.
     auto stages = [&](auto finite) __attribute__((always_inline)) {
@@ -562,7 +569,7 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
         }
     }
     // accumulator j of lane (r, g): row 8 (j / 4) + 4 g + j % 4 of the A side, column r of the B side
-    float *out = p.out + (int64_t)blockIdx.z * p.split_stride;
+    float *out = p.out + (int64_t)bz * p.split_stride;
     bf16_t *out16 = reinterpret_cast<bf16_t *>(p.out);   // bf16 outputs are never the ranges' partial matrices
     const bool o16 = p.out_bf16 != 0;
     const float scale = (EPI != FG_ADD_SCALED && EPI != FG_STORE_RBIAS) ? 0.0f
@@ -605,9 +612,17 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
             float sum = 0.0f;
 #pragma unroll
             for (int i = 0; i < 4 * G; ++i) sum += lds_all[i];
-            p.dot_part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = sum;
+            p.dot_part[(int64_t)by * gx + bx] = sum;
         }
     }
+}
+
+template <int BM, int G, int ASRC, int BSRC, int EPI, bool VEC, bool SPLIT, int AES, int BES>
+__global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kernel(FgParams p)
+{
+    __shared__ __align__(16) float lds[FgBlock<BM, G, ASRC, BSRC, VEC, SPLIT, AES, BES>::LDS];
+    __shared__ int not_finite;   // some thread's sum is an infinity or a NaN
+    f32_gemm_block<BM, G, ASRC, BSRC, EPI, VEC, SPLIT, AES, BES>(p, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, lds, not_finite);
 }
 
 // ----------------------------------------------------------------------------------------------- host side
@@ -646,24 +661,30 @@ inline FgPlan fg_room(int64_t M, int64_t N, int64_t K, int num_cus, int64_t min_
 // share a unit take `unit` us of its throughput each, a launch `base` us and every further round of blocks 2.6; outputs leave at 4.8 TB/s; adding ranges up is one more
 // launch, whose 14 TB/s say that the partial matrices come back out of the caches.  Blocks that run on a unit at a time: what
 // registers and LDS leave room for.
+struct FgKind {
+    int bm, groups, resident;
+    double chain, unit, base;
+};
+constexpr FgKind FG_KINDS[] = {{128, 1, 3, 0.51, 0.36, 5.4}, {128, 2, 1, 0.51, 0.36, 5.4}, {64, 1, 4, 0.46, 0.26, 3.7},
+                               {64, 2, 2, 0.46, 0.26, 3.7},  {64, 4, 1, 0.46, 0.26, 3.7}};
+// contraction values of each of r ranges; 0 where a range would hold nothing, or less than four stages
+inline int64_t fg_chunk(int64_t K, int r)
+{
+    const int64_t chunk = cdiv(cdiv(K, r), FG_BK) * FG_BK;
+    return r > 1 && (cdiv(K, chunk) != r || chunk < 64) ? 0 : chunk;
+}
 inline FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int max_ranges, bool groups4)
 {
-    struct Kind {
-        int bm, groups, resident;
-        double chain, unit, base;
-    };
-    static const Kind kinds[] = {{128, 1, 3, 0.51, 0.36, 5.4}, {128, 2, 1, 0.51, 0.36, 5.4}, {64, 1, 4, 0.46, 0.26, 3.7},
-                                 {64, 2, 2, 0.46, 0.26, 3.7},  {64, 4, 1, 0.46, 0.26, 3.7}};
     const bool split = f32_split_mode() != 0;
     const double out_mb = (double)M * N * 4e-6;
     FgPlan best = {128, 1, 1};
     double best_us = 1e30;
-    for (const Kind &kd : kinds) {
+    for (const FgKind &kd : FG_KINDS) {
         if (kd.groups > 1 && (!split || (kd.groups == 4 && !groups4))) continue;
         const int64_t tiles = cdiv(M, kd.bm) * cdiv(N, FG_BN);
         for (int r = 1; r <= max_ranges; ++r) {
-            const int64_t chunk = cdiv(cdiv(K, r), FG_BK) * FG_BK;
-            if (r > 1 && (cdiv(K, chunk) != r || chunk < 64)) continue;   // every range holds something, and four stages at least
+            const int64_t chunk = fg_chunk(K, r);
+            if (!chunk) continue;
             const int64_t per_cu = cdiv(tiles * r, num_cus), stages = cdiv(chunk / FG_BK, kd.groups);
             const int64_t rounds = cdiv(per_cu, kd.resident);
             const double us = kd.base + 2.6 * (rounds - 1) + stages * (rounds * kd.chain + per_cu * kd.groups * kd.unit) + out_mb * r * 0.21 +
@@ -673,6 +694,61 @@ inline FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int max_rang
                 best = {kd.bm, r, kd.groups};
             }
         }
+    }
+    return best;
+}
+// Two products side by side in one launch, blocks of one kind (rdb_f32_pair.hip).  The same model with constants of its own, fitted to
+// 14 layers of 256 to 8000 tokens ([300 .. 3001] -> [256 .. 8192], k 40 to 700), some 100 plans each: what it picks is within 5 % of
+// the backward pass of the best of them (1 % on average).  chain, unit: as above; a unit's blocks are of both products, so the mean of
+// their stages counts; out, sum: us per MB of partial matrices written, and read back; resident: bf16 matrices take less LDS.
+struct FgPairPlan {
+    int bm, groups, ranges[2];
+};
+inline FgPairPlan fg_plan_pair(const int64_t (&M)[2], const int64_t (&N)[2], const int64_t (&K)[2], int num_cus, const int (&max_ranges)[2], bool b16)
+{
+    constexpr int CAP = 64;
+    struct Kind {
+        int bm, groups;
+        double resident, chain, unit;
+    };
+    struct Model {
+        Kind kinds[3];
+        double round, out, sum, sums;
+    };
+    static const Model wide = {{{128, 1, 2, 0.438, 0.082}, {128, 2, 1, 0.375, 0.275}, {64, 2, 1, 0.074, 0.223}}, 0.34, 0.33, 0.0, 2.9};
+    static const Model narrow = {{{128, 1, 3, 0.656, 0.084}, {128, 2, 2, 0.219, 0.342}, {64, 2, 2, 0.476, 0.107}}, 0.0, 0.0, 0.29, 0.15};
+    const Model &m = b16 ? narrow : wide;
+    const double per_unit = 1.0 / num_cus;
+    FgPairPlan best = {128, 1, {1, 1}};
+    double best_us = 1e30;
+    for (const Kind &kd : m.kinds) {
+        struct Option {
+            int r;
+            double blocks, stages, out;
+        } opt[2][CAP];
+        int n[2] = {0, 0};
+        for (int i = 0; i < 2; ++i)
+            for (int r = 1; r <= max_ranges[i] && r <= CAP; ++r) {
+                const int64_t chunk = fg_chunk(K[i], r);
+                if (!chunk) continue;
+                const double mb = (double)M[i] * N[i] * 4e-6 * r;
+                opt[i][n[i]++] = {r, (double)(cdiv(M[i], kd.bm) * cdiv(N[i], FG_BN) * r), (double)cdiv(chunk / FG_BK, kd.groups), mb * (r > 1 ? m.out + m.sum : m.out)};
+            }
+        for (int i = 0; i < n[0]; ++i)
+            for (int j = 0; j < n[1]; ++j) {
+                const Option &a = opt[0][i], &b = opt[1][j];
+                const double blocks = a.blocks + b.blocks, mean = (a.blocks * a.stages + b.blocks * b.stages) / blocks, longest = a.stages > b.stages ? a.stages : b.stages;
+                // units that hold several blocks are not filled to the last one: 510 blocks in 512 places ran as two rounds
+                const double fill = blocks * per_unit, per_cu = (double)(int64_t)(fill + 0.999);
+                const double rounds = (double)(int64_t)(fill * (kd.resident > 1.0 ? 1.02 : 1.0) / kd.resident + 0.999);
+                const double alone = longest * (kd.chain + kd.groups * kd.unit);   // a unit with one block
+                const double busy = (rounds > 1.0 ? rounds * mean : longest) * kd.chain + per_cu * mean * kd.groups * kd.unit;
+                const double us = m.round * (rounds - 1.0) + (alone > busy ? alone : busy) + a.out + b.out + (a.r > 1 || b.r > 1 ? m.sums : 0.0);
+                if (us < best_us) {
+                    best_us = us;
+                    best = {kd.bm, kd.groups, {a.r, b.r}};
+                }
+            }
     }
     return best;
 }
@@ -739,15 +815,12 @@ template <int ASRC, int BSRC> struct FgGroups {
     static constexpr bool a32_b16 = BSRC == FG_KCONT;                                           // y = z . C^T, W^T = N^T . C^T
     static constexpr bool biased = ASRC == FG_KCONT && BSRC == FG_KCONT, scaled = ASRC == FG_NOISE_I || BSRC == FG_NOISE_I;
 };
-template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_t s, const char *name)
+inline bool fg_fits(const FgProduct &q)
 {
-    typedef FgGroups<ASRC, BSRC> Groups;
-    if (!q.bm) {
-        const FgPlan pl = !(Groups::scaled && q.scale) ? fg_plan(q.M, q.N, q.K, num_cus, 1, Groups::four) : fg_room(q.M, q.N, q.K, num_cus, q.K, 1);
-        q.bm = pl.bm;
-        q.groups = pl.groups;
-    }
-    if (q.a_elems >= (1ll << 29) || q.b_elems >= (1ll << 29) || q.M >= (1ll << 30) || q.N >= (1ll << 30) || q.K >= (1ll << 30)) return RDB_E_UNSUPPORTED;
+    return q.a_elems < (1ll << 29) && q.b_elems < (1ll << 29) && q.M < (1ll << 30) && q.N < (1ll << 30) && q.K < (1ll << 30) && cdiv(q.N, FG_BN) <= 65535;
+}
+inline FgParams fg_params(const FgProduct &q)
+{
     FgParams p = {};
     p.a = q.a;
     p.lda = q.lda;
@@ -774,17 +847,32 @@ template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_
     p.dotm = q.dotm;
     p.lddot = q.lddot;
     p.dot_part = q.dot_part;
-    const int splits = (int)cdiv(q.K, p.kchunk);
-    // 16-byte pieces when both matrices allow them: aligned bases and leading dimensions, and the extent along a piece a multiple of 4
-    // (along the rows of a matrix: the contraction; across them: the rows of the tile)
-    auto vec_ok = [&](int src, const float *m, int64_t ld, int64_t rows) {
+    return p;
+}
+// 16-byte pieces (8 of a bf16 matrix: four values) when both matrices allow them: aligned bases and leading dimensions, and the extent
+// along a piece a multiple of 4 (along the rows of a matrix: the contraction; across them: the rows of the tile)
+inline bool fg_vec(const FgProduct &q, int asrc, int bsrc)
+{
+    auto ok = [&](int src, const float *m, int64_t ld, int64_t rows) {
         if (src != FG_KCONT && src != FG_MCONT) return true;
         return fg_aligned16(m) && ld % 4 == 0 && (src == FG_KCONT ? q.K % 4 == 0 : rows % 4 == 0);
     };
-    const bool vec = vec_ok(ASRC, q.a, q.lda, q.M) && vec_ok(BSRC, q.b, q.ldb, q.N);   // bf16 matrices: 8-byte pieces of four values
+    return ok(asrc, q.a, q.lda, q.M) && ok(bsrc, q.b, q.ldb, q.N);
+}
+template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_t s, const char *name)
+{
+    typedef FgGroups<ASRC, BSRC> Groups;
+    if (!q.bm) {
+        const FgPlan pl = !(Groups::scaled && q.scale) ? fg_plan(q.M, q.N, q.K, num_cus, 1, Groups::four) : fg_room(q.M, q.N, q.K, num_cus, q.K, 1);
+        q.bm = pl.bm;
+        q.groups = pl.groups;
+    }
+    if (!fg_fits(q)) return RDB_E_UNSUPPORTED;
+    const FgParams p = fg_params(q);
+    const int splits = (int)cdiv(q.K, p.kchunk);
+    const bool vec = fg_vec(q, ASRC, BSRC);
     const bool a16 = (ASRC == FG_KCONT || ASRC == FG_MCONT) && q.a_es == 2, b16 = (BSRC == FG_KCONT || BSRC == FG_MCONT) && q.b_es == 2;
     if (q.split && ((a16 && b16) ? !Groups::a16_b16 : a16 ? !Groups::a16_b32 : b16 && !Groups::a32_b16)) return RDB_E_UNSUPPORTED;
-    if (cdiv(q.N, FG_BN) > 65535) return RDB_E_UNSUPPORTED;   // the grid's y
     const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)splits);
     auto run = [&](auto epi_) {
         constexpr int EPI = decltype(epi_)::value;

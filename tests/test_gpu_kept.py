@@ -75,3 +75,28 @@ def test_few_token_forward_and_dx_on_the_matrix_cores(T, in_f, out_f, k):
     rc = _lib.load().rdb_linear_fwd(y.data_ptr(), out_f, xc.data_ptr(), in_f, cc.data_ptr(), None, None, ctypes.byref(d), None, 0,
                                     torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and _rel(y, x.double() @ W.t()) < 5e-6
+
+
+# every kind of block the pair of products in one launch is planned for (128 rows with one group and with two, 64 rows with two), with
+# one and with several ranges on either side, whole and ragged tiles, pieces of four that are and are not aligned
+@pytest.mark.parametrize("T,in_f,out_f,k,dtype", [(131, 259, 129, 65, torch.float32), (131, 259, 129, 65, torch.bfloat16), (2048, 768, 3072, 256, torch.float32),
+                                                  (902, 720, 886, 606, torch.float32), (1552, 484, 2592, 20, torch.float32), (1000, 2001, 4000, 150, torch.bfloat16),
+                                                  (6000, 700, 3001, 333, torch.bfloat16), (3000, 130, 257, 65, torch.bfloat16), (300, 2048, 2048, 512, torch.float32)])
+def test_both_products_over_dy_in_one_launch(T, in_f, out_f, k, dtype):
+    """dx and dC of one backward call, where t = dy . C and dC = dy^T . z share a launch, against float64, against the calls that want only
+    one of them, and bit for bit run to run."""
+    print(f"case pair T={T} in={in_f} out={out_f} k={k} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(T + k)
+    x, dy = torch.randn(T, in_f, generator=g).to(dtype), torch.randn(T, out_f, generator=g).to(dtype)
+    c = (torch.randn(out_f, k, generator=g) / k ** 0.5).to(dtype)
+    N = ops.sq5_gen_2d(in_f, k, 8).double().cpu()
+    leaves = [x.cuda().requires_grad_(), c.cuda().requires_grad_()]
+    y = ops.linear(leaves[0], leaves[1], in_f, out_f, in_f, 1, 8, None, None)
+    dx, dc = torch.autograd.grad(y, leaves, dy.cuda(), retain_graph=True)
+    D = dy.double()
+    tol = 5e-6 if dtype == torch.float32 else 2.0**-9   # fp32 sums throughout; bf16 results are rounded once
+    assert _rel(dx, (D @ c.double()) @ N.t()) < tol and _rel(dc, D.t() @ (x.double() @ N)) < tol
+    again = torch.autograd.grad(y, leaves, dy.cuda(), retain_graph=True)
+    assert torch.equal(dx, again[0]) and torch.equal(dc, again[1])
+    assert _rel(torch.autograd.grad(y, leaves[:1], dy.cuda(), retain_graph=True)[0], dx.double().cpu()) < 2 * tol
+    assert _rel(torch.autograd.grad(y, leaves[1:], dy.cuda())[0], dc.double().cpu()) < 2 * tol

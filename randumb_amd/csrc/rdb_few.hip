@@ -1,0 +1,596 @@
+// Forward pass of a matrix-coef layer for a handful of tokens (a served model generating): z = x . N^T, y = z . C^T (+ bias) on the
+// matrix cores with 16 x 16 tiles, at fp32 accuracy whatever the operands' type, in one launch.
+//
+// What bounds it is latency: 16 tokens x 4096 -> 11008, k = 256 move 6 MB and multiply next to nothing.  Contracting blocks (16 coefficients
+// x a chunk of in_f, the tokens all at once, so that every noise value is hashed once) leave partial sums of z; expanding blocks (64
+// output features) have their rows of C in registers by the time these are there, add them up in chunk order, and multiply.  In
+// one launch the contracting blocks come first and publish a tag each (rdb_common.hpp); where the partial sums are so many that
+// reading them around the dies' L2 caches costs more than a launch, the two kinds of block are two launches of the same kernel.
+// us per call, three launches on the vector ALU (or the kernels for many tokens) -> here: 16 tokens x 4096 -> 11008, k = 256, bf16 14.5 ->
+// 11.5; 1 x 7512 -> 2376, k = 512, bf16 34.6 -> 14.0; 5 x 1001 -> 999, k = 99, bf16 17.1 -> 7.5; 22 x 264 -> 352, k = 64, fp32 17.7 -> 8.6;
+// 1 x 4096 -> 4096, k = 16, fp32 9.0 -> 8.6.  What is left is launches and memory round trips: x in, partial sums out and in, y out.
+//
+// fp32 accuracy: a noise value is exactly three bf16 parts, so its products with bf16 activations are exact in three matrix instructions;
+// so are those of z (fp32) with bf16 coefficients.  fp32 activations and coefficients are split as well: the six largest of the nine
+// products (rdb_f32.hpp says what is left out).  Infinities come out as they do of fp32 products: an infinite fp32 value is split into
+// (largest, largest, infinity), an infinite bf16 value meets its partner's lower parts as the largest finite one, and sums of y that
+// are not finite are done again with parts of one sign.
+#include "rdb_common.hpp"
+#include <algorithm>
+#include <type_traits>
+
+namespace rdb {
+
+
+constexpr int FEW_ROWS = 64;       // output features of an expanding block: 16 a wave
+constexpr int FEW_COEFS = 16;      // coefficients of a contracting block
+constexpr int FEW_STEPS = 4;       // steps of 32 contraction values a contracting wave hashes ahead of its products
+constexpr int FEW_TOKENS = 48, FEW_K = 512;   // z's three parts in LDS: at most 150 KB
+
+struct FewParams {
+    void *y;
+    const void *x, *coef, *bias;
+    int64_t ldx, ldy;
+    float *part;   // [chunks][ranges of 16 coefficients][tokens][16]
+    int T, in_f, out_f, k, chunks, ranges;
+    int wave_values;     // contraction values per wave and chunk: a multiple of 32
+    int x_vec, c_vec, y_vec;   // 16-byte pieces of x and C, 4 values of y at a time
+    uint32_t seed;
+    int c_blocks;        // contracting blocks of this launch: they come first
+    unsigned long long *slots;   // NULL, or one tag per contracting block
+    unsigned long long tag;
+    SyncWait wait;
+    unsigned int *count;
+    int consumers;
+};
+
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+
+// eight values as three bf16 fragments
+struct Split8 {
+    bf16x8 h, m, l;
+};
+__device__ __forceinline__ void few_split2(float v0, float v1, uint32_t &h, uint32_t &m, uint32_t &l)
+{
+    constexpr float top = 3.3895313892515355e38f;   // the largest bf16: nothing below an infinity rounds to one
+    h = f32x2_to_bf16x2(__builtin_amdgcn_fmed3f(v0, -top, top), __builtin_amdgcn_fmed3f(v1, -top, top));
+    v0 -= __uint_as_float(h << 16);
+    v1 -= __uint_as_float(h & 0xffff0000u);
+    m = f32x2_to_bf16x2(__builtin_amdgcn_fmed3f(v0, -top, top), __builtin_amdgcn_fmed3f(v1, -top, top));
+    l = f32x2_to_bf16x2(v0 - __uint_as_float(m << 16), v1 - __uint_as_float(m & 0xffff0000u));
+}
+__device__ __forceinline__ Split8 few_split8(const f32x8 &v)
+{
+    u32x4_t h, m, l;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        uint32_t a, b, c;
+        few_split2(v[2 * e], v[2 * e + 1], a, b, c);
+        h[e] = a;
+        m[e] = b;
+        l[e] = c;
+    }
+    return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
+}
+// The same with the parts cut off and not rounded, all of one sign: no two of a product's terms overflow to different sides.  What is
+// left out of a product of two such splits is up to 2^-21 of it and of its sign, so only sums that came out not finite are done with it.
+__device__ __forceinline__ Split8 few_split8_any(const f32x8 &v)
+{
+    constexpr float top = 3.40282346638528859812e38f;
+    u32x4_t p[3];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float rest = v[e];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const uint32_t part = __float_as_uint(q < 2 ? __builtin_amdgcn_fmed3f(rest, -top, top) : rest) & 0xffff0000u;
+            rest -= __uint_as_float(part);
+            p[q][e / 2] = e & 1 ? p[q][e / 2] | part : part >> 16;
+        }
+    }
+    return {__builtin_bit_cast(bf16x8, p[0]), __builtin_bit_cast(bf16x8, p[1]), __builtin_bit_cast(bf16x8, p[2])};
+}
+// eight values back from their parts (exactly)
+__device__ __forceinline__ f32x8 few_join8(const Split8 &z)
+{
+    const u32x4_t h = __builtin_bit_cast(u32x4_t, z.h), m = __builtin_bit_cast(u32x4_t, z.m), l = __builtin_bit_cast(u32x4_t, z.l);
+    f32x8 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[2 * e] = (__uint_as_float(h[e] << 16) + __uint_as_float(m[e] << 16)) + __uint_as_float(l[e] << 16);
+        v[2 * e + 1] = (__uint_as_float(h[e] & 0xffff0000u) + __uint_as_float(m[e] & 0xffff0000u)) + __uint_as_float(l[e] & 0xffff0000u);
+    }
+    return v;
+}
+// infinities as the largest finite value of their sign, for the products with the lower parts of the other side
+__device__ __forceinline__ bf16x8 few_finite(const bf16x8 &v)
+{
+    u32x4_t w = __builtin_bit_cast(u32x4_t, v);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t lo = w[e] & 0x7fffu, hi = (w[e] >> 16) & 0x7fffu;
+        w[e] = (w[e] & 0x80008000u) | min(lo, 0x7f7fu) | (min(hi, 0x7f7fu) << 16);
+    }
+    return __builtin_bit_cast(bf16x8, w);
+}
+__device__ __forceinline__ f32x4 few_mma(const bf16x8 &a, const bf16x8 &b, const f32x4 &c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+
+// Eight consecutive values of a row as they are in memory; a fragment lane's share of a matrix operand
+template <typename E> struct FewRaw;
+template <> struct FewRaw<bf16_t> {
+    u32x4_t w;
+};
+template <> struct FewRaw<float> {
+    f32x4 lo, hi;
+};
+// values at .. at + 7 of the row at `row`, zeros from n on and where !ok
+template <typename E> __device__ __forceinline__ FewRaw<E> few_load(const E *row, int at, int n, bool ok, int vec)
+{
+    FewRaw<E> r;
+    if (vec) {   // n is a multiple of 8: a piece lies inside or outside
+        const bool in = ok && at < n;
+        const E *src = in ? row + at : row;
+        if constexpr (sizeof(E) == 2) {
+            r.w = *reinterpret_cast<const u32x4_t *>(src);
+            if (!in) r.w = u32x4_t{0, 0, 0, 0};
+        } else {
+            r.lo = *reinterpret_cast<const f32x4 *>(src);
+            r.hi = *reinterpret_cast<const f32x4 *>(src + 4);
+            if (!in) r.lo = r.hi = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        return r;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const bool in = ok && at + e < n;
+        const E v = row[in ? at + e : 0];
+        if constexpr (sizeof(E) == 2) {
+            const uint32_t b = in ? (uint32_t)v << (16 * (e & 1)) : 0u;
+            r.w[e / 2] = e & 1 ? r.w[e / 2] | b : b;
+        } else {
+            (e < 4 ? r.lo : r.hi)[e & 3] = in ? v : 0.0f;
+        }
+    }
+    return r;
+}
+
+// acc (the large products) and low (the small ones) += A . B^T, A from memory, B in three parts
+template <typename E> struct FewSide;
+template <> struct FewSide<bf16_t> {
+    bf16x8 v, f;
+    template <bool ANY = false> __device__ __forceinline__ void set(const FewRaw<bf16_t> &r)
+    {
+        v = __builtin_bit_cast(bf16x8, r.w);
+        f = few_finite(v);
+    }
+    // the side from memory as the A operand (rows of the result)
+    __device__ __forceinline__ void mma_a(f32x4 &acc, f32x4 &low, const Split8 &b) const
+    {
+        low = few_mma(f, b.l, low);
+        low = few_mma(f, b.m, low);
+        acc = few_mma(v, b.h, acc);
+    }
+};
+template <> struct FewSide<float> {
+    Split8 s;
+    template <bool ANY = false> __device__ __forceinline__ void set(const FewRaw<float> &r)
+    {
+        const f32x8 v = {r.lo[0], r.lo[1], r.lo[2], r.lo[3], r.hi[0], r.hi[1], r.hi[2], r.hi[3]};
+        s = ANY ? few_split8_any(v) : few_split8(v);
+    }
+    __device__ __forceinline__ void mma_a(f32x4 &acc, f32x4 &low, const Split8 &b) const
+    {
+        low = few_mma(s.m, b.m, low);
+        low = few_mma(s.l, b.h, low);
+        low = few_mma(s.h, b.l, low);
+        low = few_mma(s.m, b.h, low);
+        low = few_mma(s.h, b.m, low);
+        acc = few_mma(s.h, b.h, acc);
+    }
+};
+
+// Block (range, chunk): z[all tokens][16 coefficients] over the chunk, a quarter of it to a wave.
+template <typename E, int TT> __device__ __forceinline__ void few_contract(const FewParams &p, int b, float *__restrict__ lds)
+{
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const int range = b % p.ranges, ch = b / p.ranges, m = range * FEW_COEFS + r;
+    const int i_begin = (ch * 4 + wave) * p.wave_values;
+    const E *const x = static_cast<const E *>(p.x);
+    const E *row[TT];
+    bool live[TT];
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+        live[tt] = tt * 16 + r < p.T;
+        row[tt] = x + (int64_t)(live[tt] ? tt * 16 + r : 0) * p.ldx;
+    }
+    f32x4 acc[TT], low[TT];
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) acc[tt] = low[tt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i0 = 0; i0 < p.wave_values; i0 += 32 * FEW_STEPS) {
+        FewRaw<E> raw[FEW_STEPS];
+        auto request = [&](int tt) {
+#pragma unroll
+            for (int s = 0; s < FEW_STEPS; ++s)
+                if (i0 + s * 32 < p.wave_values) raw[s] = few_load<E>(row[tt], i_begin + i0 + s * 32 + g * 8, p.in_f, live[tt], p.x_vec);
+        };
+        request(0);
+        // values past in_f meet zeros of x
+        Split8 noise[FEW_STEPS];
+#pragma unroll
+        for (int s = 0; s < FEW_STEPS; ++s)
+            if (i0 + s * 32 < p.wave_values) {
+                const uint32_t first = sq5_first((uint32_t)(i_begin + i0 + s * 32 + g * 8), (uint32_t)m, p.seed);
+                f32x8 v;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = sq5_unit(sq5_tail(first + (uint32_t)e * PN1));
+                noise[s] = few_split8(v);
+            }
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) {
+            if (tt * 16 >= p.T) break;   // uniform
+            FewSide<E> a[FEW_STEPS];
+#pragma unroll
+            for (int s = 0; s < FEW_STEPS; ++s)
+                if (i0 + s * 32 < p.wave_values) a[s].set(raw[s]);
+            if (tt + 1 < TT && (tt + 1) * 16 < p.T) request(tt + 1);
+#pragma unroll
+            for (int s = 0; s < FEW_STEPS; ++s)
+                if (i0 + s * 32 < p.wave_values) a[s].mma_a(acc[tt], low[tt], noise[s]);
+        }
+    }
+    // result element j of lane (r, g): token 4 g + j, coefficient r; the waves' sums meet in LDS
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) lds[((wave * TT + tt) * 16 + g * 4 + j) * 16 + r] = acc[tt][j] + low[tt][j];
+    __syncthreads();
+    float *const out = p.part + (int64_t)(ch * p.ranges + range) * p.T * 16;
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+        const int t = tt * 16 + (tid >> 4);
+        if (t < p.T) {
+            float v = lds[tt * 256 + tid];
+#pragma unroll
+            for (int w = 1; w < 4; ++w) v += lds[(w * TT + tt) * 256 + tid];
+            __hip_atomic_store(out + (int64_t)t * 16 + (tid & 15), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+
+// Block: 64 output features, all tokens.
+template <typename E, int KS, int TT> __device__ __forceinline__ void few_expand(const FewParams &p, int b, unsigned char *__restrict__ smem)
+{
+    constexpr int KW = KS * 32, LD = KW + 8;   // 16 bytes of padding: 16 rows' pieces lie in different banks
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const int o0 = b * FEW_ROWS + wave * 16;
+    bf16_t *const planes = reinterpret_cast<bf16_t *>(smem);
+    const int PLANE = (p.T + 15) / 16 * 16 * LD;
+    E *const y = static_cast<E *>(p.y);
+    // the wave's rows of C, before anything is waited for
+    FewRaw<E> c[KS];
+    {
+        const bool ok = o0 + r < p.out_f;
+        const E *const row = static_cast<const E *>(p.coef) + (int64_t)(ok ? o0 + r : 0) * p.k;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) c[s] = few_load<E>(row, s * 32 + g * 8, p.k, ok, p.c_vec);
+    }
+    if (p.slots) {
+        __shared__ int verdict;
+        const int n = p.chunks * p.ranges;
+        if (tid < 64) {
+            bool there = false;
+            for (int it = 0; it < p.wait.polls && !there; ++it) {
+                bool mine = true;
+                for (int i = lane; i < n; i += 64) mine &= __hip_atomic_load(p.slots + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == p.tag;
+                there = __all(mine);
+                if (!there) __builtin_amdgcn_s_sleep(10);
+            }
+            if (there) {   // the last of the consumers clears the slots (a recorded launch runs again with the same tag)
+                unsigned int old = 0;
+                if (lane == 0) old = __hip_atomic_fetch_add(p.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                old = (unsigned int)__builtin_amdgcn_readfirstlane((int)old);
+                if (old == (unsigned int)(p.consumers - 1))
+                    for (int i = lane; i < n; i += 64) __hip_atomic_store(p.slots + i, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            } else if (lane == 0) {
+                if (p.wait.err) atomicOr(p.wait.err, 2u);
+                atomicAdd(p.wait.giveups, 1u);
+            }
+            if (tid == 0) verdict = there ? 1 : 0;
+        }
+        __syncthreads();
+        if (verdict == 0) {   // gave up: the block's share of the output becomes NaN, never a sum of whatever is in memory
+            for (int i = tid; i < p.T * FEW_ROWS; i += 256) {
+                const int t = i / FEW_ROWS, o = b * FEW_ROWS + i % FEW_ROWS;
+                if (o < p.out_f) elem<E>::store(y + (int64_t)t * p.ldy + o, __uint_as_float(0x7fc00000u));
+            }
+            return;
+        }
+    }
+    // z: four coefficients of a token at a time, the chunks' sums in chunk order, then its three parts
+    const int n4 = p.ranges * p.T * 4;
+    const int64_t stride = (int64_t)p.ranges * p.T * 16;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(p.part, 0, (int)(stride * p.chunks * 4), 0x00020000);
+    // IB entries of CB chunks in flight
+    auto add_up = [&](auto ib_, auto cb_) __attribute__((always_inline)) {
+        constexpr int IB = decltype(ib_)::value, CB = decltype(cb_)::value;
+        for (int i0 = tid; i0 < n4; i0 += 256 * IB) {
+            f32x4 v[IB];
+            for (int c0 = 0; c0 < p.chunks; c0 += CB) {
+                f32x4 u[IB][CB];
+#pragma unroll
+                for (int i = 0; i < IB; ++i)
+#pragma unroll
+                    for (int q = 0; q < CB; ++q) {
+                        const int at = (int)(((int64_t)min(c0 + q, p.chunks - 1) * stride + (int64_t)min(i0 + i * 256, n4 - 1) * 4) * 4);
+                        u[i][q] = __builtin_bit_cast(f32x4, p.slots ? __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, SCOPE_DEVICE) : __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
+                    }
+#pragma unroll
+                for (int i = 0; i < IB; ++i)
+#pragma unroll
+                    for (int q = 0; q < CB; ++q) {
+                        if (c0 + q >= p.chunks) continue;
+                        v[i] = c0 + q == 0 ? u[i][q] : v[i] + u[i][q];
+                    }
+            }
+#pragma unroll
+            for (int i = 0; i < IB; ++i) {
+                const int e = i0 + i * 256;
+                if (e >= n4) continue;
+                const int rt = e >> 2, range = rt / p.T, t = rt - range * p.T, m = range * FEW_COEFS + (e & 3) * 4;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (m + j >= p.k) v[i][j] = 0.0f;
+                uint2 h, mm, l;
+                few_split2(v[i][0], v[i][1], h.x, mm.x, l.x);
+                few_split2(v[i][2], v[i][3], h.y, mm.y, l.y);
+                bf16_t *const dst = planes + t * LD + m;
+                *reinterpret_cast<uint2 *>(dst) = h;
+                *reinterpret_cast<uint2 *>(dst + PLANE) = mm;
+                *reinterpret_cast<uint2 *>(dst + 2 * PLANE) = l;
+            }
+        }
+    };
+    if (p.chunks == 1) add_up(std::integral_constant<int, 16>{}, std::integral_constant<int, 1>{});
+    else if (p.chunks <= 4) add_up(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
+    else add_up(std::integral_constant<int, 2>{}, std::integral_constant<int, 8>{});
+    // coefficients beyond the last range meet zeros of C: they must be finite
+    const int tail4 = (KW - p.ranges * FEW_COEFS) / 4;
+    if (tail4 > 0)
+        for (int e = tid; e < 3 * p.T * tail4; e += 256) {
+            const int row = e / tail4, pl = row / p.T;
+            *reinterpret_cast<uint2 *>(planes + pl * PLANE + (row - pl * p.T) * LD + p.ranges * FEW_COEFS + (e - row * tail4) * 4) = make_uint2(0u, 0u);
+        }
+    __syncthreads();
+    f32x4 acc[TT], low[TT];
+    auto product = [&](auto any) __attribute__((always_inline)) {
+        constexpr bool ANY = decltype(any)::value;
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) acc[tt] = low[tt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            if (s * 32 >= p.k) break;   // uniform
+            FewSide<E> a;
+            a.template set<ANY>(c[s]);
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) {
+                if (tt * 16 >= p.T) break;
+                const bf16_t *const src = planes + (tt * 16 + r) * LD + s * 32 + g * 8;   // tokens from T on: whatever lies there, in columns nobody stores
+                Split8 z = {*reinterpret_cast<const bf16x8 *>(src), *reinterpret_cast<const bf16x8 *>(src + PLANE), *reinterpret_cast<const bf16x8 *>(src + 2 * PLANE)};
+                if (ANY) z = few_split8_any(few_join8(z));
+                a.mma_a(acc[tt], low[tt], z);
+            }
+        }
+    };
+    product(std::false_type{});
+    float zero = 0.0f;   // stays so as long as every sum is finite
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) zero = tt * 16 + r < p.T ? fmaf(acc[tt][j] + low[tt][j], 0.0f, zero) : zero;
+    if (__any(zero != 0.0f)) product(std::true_type{});
+    // result element j of lane (r, g): output feature o0 + 4 g + j, token r
+    const int o = o0 + g * 4;
+    float bv[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bv[j] = p.bias && o + j < p.out_f ? elem<E>::load(static_cast<const E *>(p.bias) + o + j) : 0.0f;
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+        const int t = tt * 16 + r;
+        if (t >= p.T || o >= p.out_f) continue;
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = acc[tt][j] + low[tt][j] + bv[j];
+        E *const dst = y + (int64_t)t * p.ldy + o;
+        if (p.y_vec) {   // out_f is a multiple of 4
+            if constexpr (sizeof(E) == 2) *reinterpret_cast<uint2 *>(dst) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));
+            else *reinterpret_cast<f32x4 *>(dst) = f32x4{v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (o + j < p.out_f) elem<E>::store(dst + j, v[j]);
+        }
+    }
+}
+
+// the chunks' sums, in chunk order, into chunk 0's place
+__global__ __launch_bounds__(256) void few_sum_kernel(float *__restrict__ part, int64_t n4, int chunks)
+{
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= n4) return;
+    f32x4 *const at = reinterpret_cast<f32x4 *>(part) + e;
+    f32x4 v = *at;
+    for (int c0 = 1; c0 < chunks; c0 += 8) {
+        f32x4 u[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) u[q] = at[(int64_t)min(c0 + q, chunks - 1) * n4];
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            if (c0 + q < chunks) v += u[q];
+    }
+    *at = v;
+}
+
+template <typename E, int KS, int TT> __global__ __launch_bounds__(256, 1) void few_fwd_kernel(FewParams p)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int b = blockIdx.x;
+    if (b >= p.c_blocks) {
+        few_expand<E, KS, TT>(p, b - p.c_blocks, smem);
+        return;
+    }
+    if (p.slots && threadIdx.x == 0) __hip_atomic_store(p.slots + b, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // a replay may find its tag
+    few_contract<E, TT>(p, b, reinterpret_cast<float *>(smem));
+    if (!p.slots) return;
+    if (b == 0 && threadIdx.x == 0) __hip_atomic_store(p.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    publish_tag(p.slots + b, p.tag);
+}
+
+// ----------------------------------------------------------------------------------------------- host side
+// Where these kernels are ahead of those of rdb_smallk.hip, rdb_factored.hip and rdb_f32.hip (us per call, before -> here): bf16 up to 48
+// tokens (40 x 8192 -> 8192, k = 64: 20.5 -> 15.6; 64 x 768 -> 3072, k = 256: 14.6 -> 17.6); fp32, six products instead of three,
+// up to 48 tokens with k <= 64 (48 x 1384 -> 3328, k = 32: 14.2 -> 12.3), 32 with k <= 128 (32 x 2048 -> 2048, k = 128: 13.0 -> 11.2), 16
+// with k <= 256 (24 x 4096 -> 4096, k = 256: 14.6 -> 16.0), and again 32 beyond, where the others have no kernel for few tokens.
+// The factored form is taken as far as everywhere: up to 16 times the products of one with a stored weight.
+static bool few_ok(const rdb_linear_desc *d)
+{
+    const bool f32 = d->act_dtype == RDB_F32 && d->coef_dtype == RDB_F32, b16 = d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16;
+    const int most = b16 || d->k <= 64 ? FEW_TOKENS : d->k <= 128 || d->k > 256 ? 32 : 16;
+    return (f32 || b16) && d->algo == RDB_ALGO_AUTO && d->coef_rows != 0 && d->k > 0 && d->k <= FEW_K && d->tokens > 0 && d->tokens <= most && d->in_f > 0 &&
+           d->out_f > 0 && d->in_f < (1 << 20) && d->out_f < (1 << 24) && d->k * (d->in_f + d->out_f) < 16 * d->in_f * d->out_f;
+}
+// Chunks: about eight of them (sixteen where there is one range of coefficients), of 128 to 512 values (a contracting block hashes a chunk for 16 coefficients: 128 values cost it 0.6 us;
+// an expanding block reads eight at a time: 1 x 4096 -> 4096, k = 16: chunks of 128, 256, 512, 1024: 8.9, 8.0, 8.2, 10.9 us).
+// sum: beyond 200 KB of partial sums they are added up once, by a launch of its own, and not by every expanding block
+// (32 tokens x 4096 -> 11008, k = 256: 15.6 -> 14.9 us; 16 tokens, 131 KB: 11.5, and 12.7 with it).
+// one: a single launch where the expanding blocks are few and the partial sums small; tags and reads that go around L2 cost many
+// blocks more than a launch does (5 x 1001 -> 999, k = 99: two launches 9.2, one 7.5; 16 x 4096 -> 11008, k = 256: 11.5 and 13.5; 1 x 4096
+// -> 4096, k = 16: 8.0 and 8.6, but a program's host takes 10.7 to issue two).
+struct FewPlan {
+    int wave_values, chunks, ranges;
+    bool sum, one;
+    int64_t part_bytes;
+};
+static FewPlan few_plan(const rdb_linear_desc *d)
+{
+    FewPlan f;
+    f.ranges = (int)cdiv(d->k, FEW_COEFS);
+    int64_t chunk = 128;
+    while (chunk < 512 && chunk * (f.ranges == 1 ? 16 : 8) < d->in_f) chunk *= 2;
+    const int64_t per_chunk = (int64_t)f.ranges * d->tokens * FEW_COEFS * 4;
+    f.sum = cdiv(d->in_f, chunk) * per_chunk > 200 * 1024;
+    if (f.sum && chunk > 256) chunk = 256;
+    f.wave_values = (int)chunk / 4;
+    f.chunks = (int)cdiv(d->in_f, chunk);
+    f.part_bytes = f.chunks * per_chunk;
+    const int64_t e_blocks = cdiv(d->out_f, FEW_ROWS);
+    f.one = !f.sum && ((e_blocks <= 32 && f.part_bytes <= 100 * 1024) || (e_blocks <= 80 && f.part_bytes <= 32 * 1024));
+    return f;
+}
+
+int64_t linear_few_workspace(const rdb_linear_desc *d)
+{
+    if (!few_ok(d)) return 0;
+    const FewPlan f = few_plan(d);
+    return f.part_bytes + (int64_t)f.chunks * f.ranges * 8 + 8;   // ... the tags, and the consumers' counter
+}
+
+template <typename E, int KS, int TT> static int few_launch(FewParams p, int c_blocks, int e_blocks, bool one, bool sum, hipStream_t s)
+{
+    const size_t smem_z = (size_t)4 * TT * 1024, smem_y = (size_t)3 * cdiv(p.T, 16) * 16 * (KS * 32 + 8) * 2, smem = std::max(smem_z, smem_y);
+    const auto kernel = few_fwd_kernel<E, KS, TT>;
+    if (int rc = reserve_lds(reinterpret_cast<const void *>(kernel), smem, "few_fwd_kernel")) return rc;
+    p.c_blocks = c_blocks;
+    if (one) {
+        kernel<<<(unsigned)(c_blocks + e_blocks), 256, smem, s>>>(p);
+        return check_launch("few_fwd_kernel");
+    }
+    kernel<<<(unsigned)c_blocks, 256, smem_z, s>>>(p);
+    if (int rc = check_launch("few_fwd_kernel (z)")) return rc;
+    if (sum) {
+        const int64_t n4 = (int64_t)p.ranges * p.T * 4;
+        few_sum_kernel<<<(unsigned)cdiv(n4, 256), 256, 0, s>>>(p.part, n4, p.chunks);
+        if (int rc = check_launch("few_sum_kernel")) return rc;
+        p.chunks = 1;
+    }
+    p.c_blocks = 0;
+    kernel<<<(unsigned)e_blocks, 256, smem_y, s>>>(p);
+    return check_launch("few_fwd_kernel (y)");
+}
+template <typename E> static int few_dispatch(const FewParams &p, int c_blocks, int e_blocks, bool one, bool sum, hipStream_t s)
+{
+    const int tt = (p.T + 15) / 16;
+    auto of = [&](auto ks_) {
+        constexpr int KS = decltype(ks_)::value;
+        if (tt == 1) return few_launch<E, KS, 1>(p, c_blocks, e_blocks, one, sum, s);
+        if (tt == 2) return few_launch<E, KS, 2>(p, c_blocks, e_blocks, one, sum, s);
+        return few_launch<E, KS, 3>(p, c_blocks, e_blocks, one, sum, s);
+    };
+    if (p.k <= 128) return of(std::integral_constant<int, 4>{});
+    if (p.k <= 256) return of(std::integral_constant<int, 8>{});
+    return of(std::integral_constant<int, 16>{});
+}
+
+static FewParams few_params(const rdb_linear_desc *d, const FewPlan &f, void *y, int64_t ldy, const void *x, int64_t ldx, const void *coef, const void *bias,
+                            void *workspace)
+{
+    const int es = d->act_dtype == RDB_BF16 ? 2 : 4;
+    FewParams p = {};
+    p.y = y;
+    p.x = x;
+    p.coef = coef;
+    p.bias = bias;
+    p.ldx = ldx;
+    p.ldy = ldy;
+    p.part = static_cast<float *>(workspace);
+    p.T = (int)d->tokens;
+    p.in_f = (int)d->in_f;
+    p.out_f = (int)d->out_f;
+    p.k = (int)d->k;
+    p.chunks = f.chunks;
+    p.ranges = f.ranges;
+    p.wave_values = f.wave_values;
+    p.x_vec = d->in_f % 8 == 0 && ldx * es % 16 == 0 && ((uintptr_t)x & 15) == 0;
+    p.c_vec = d->k % 8 == 0 && ((uintptr_t)coef & 15) == 0;
+    p.y_vec = d->out_f % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)y & (4 * es - 1)) == 0;
+    p.seed = d->seed;
+    return p;
+}
+static int few_tags(FewParams &p, const FewPlan &f, int e_blocks, int polls)
+{
+    p.slots = reinterpret_cast<unsigned long long *>(reinterpret_cast<char *>(p.part) + f.part_bytes);
+    p.tag = next_sync_tag();
+    p.wait = {nullptr, nullptr, polls};
+    p.count = reinterpret_cast<unsigned int *>(p.slots + (int64_t)f.chunks * f.ranges);
+    p.consumers = e_blocks;
+    return sync_giveups_ptr(&p.wait.giveups);
+}
+
+// Returns RDB_E_UNSUPPORTED, without setting an error, when the request does not fit.
+int linear_fwd_few(void *y, int64_t ldy, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias, const rdb_linear_desc *d,
+                   void *workspace, int64_t workspace_bytes, hipStream_t s)
+{
+    if (scale_bias || !few_ok(d) || !workspace || ((uintptr_t)workspace & 15) || workspace_bytes < linear_few_workspace(d)) return RDB_E_UNSUPPORTED;
+    const FewPlan f = few_plan(d);
+    FewParams p = few_params(d, f, y, ldy, x, ldx, coef, bias, workspace);
+    const int c_blocks = f.chunks * f.ranges, e_blocks = (int)cdiv(d->out_f, FEW_ROWS);
+    const bool one = f.one && one_launch_mode();
+    if (one) {
+        if (int rc = few_tags(p, f, e_blocks, SYNC_SPIN_LIMIT)) return rc;
+    }
+    return d->act_dtype == RDB_BF16 ? few_dispatch<bf16_t>(p, c_blocks, e_blocks, one, f.sum, s) : few_dispatch<float>(p, c_blocks, e_blocks, one, f.sum, s);
+}
+
+// Test hook: only the expanding blocks of the one-launch form, waiting (at most `polls` polls each) for tags that nobody publishes.
+int selftest_giveup_few(void *y, int64_t ldy, const void *coef, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, int polls, hipStream_t s)
+{
+    if (!few_ok(d) || ((uintptr_t)workspace & 15) || workspace_bytes < linear_few_workspace(d)) return RDB_E_UNSUPPORTED;
+    const FewPlan f = few_plan(d);
+    if (!f.one) return RDB_E_UNSUPPORTED;
+    FewParams p = few_params(d, f, y, ldy, nullptr, 0, coef, nullptr, workspace);
+    const int e_blocks = (int)cdiv(d->out_f, FEW_ROWS);
+    if (int rc = few_tags(p, f, e_blocks, polls)) return rc;
+    return d->act_dtype == RDB_BF16 ? few_dispatch<bf16_t>(p, 0, e_blocks, true, false, s) : few_dispatch<float>(p, 0, e_blocks, true, false, s);
+}
+
+}  // namespace rdb

@@ -340,6 +340,10 @@ int64_t linear_bwd_projected_workspace(const rdb_linear_desc *d, int num_cus, bo
 int linear_dx_factored(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *coef, const void *scale_bias,
                        const rdb_linear_desc *d, int num_cus, void *workspace, int64_t workspace_bytes, hipStream_t s);
 
+// rdb_few.hip
+int linear_fwd_few(void *y, int64_t ldy, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias, const rdb_linear_desc *d,
+                   void *workspace, int64_t workspace_bytes, hipStream_t s);
+int64_t linear_few_workspace(const rdb_linear_desc *d);
 // rdb_big.hip
 void set_big_tiles_mode(int mode);
 int big_tiles_mode();
@@ -443,6 +447,7 @@ extern "C" int64_t rdb_linear_workspace_bytes(int op, const rdb_linear_desc *d)
         const int64_t few = linear_smallk_workspace(&dd);
         if (few > need) need = few;
     }
+    if (op == RDB_OP_LINEAR_FWD) need = std::max(need, linear_few_workspace(d));
     return need;
 }
 
@@ -506,6 +511,10 @@ extern "C" int rdb_linear_fwd(void *y, int64_t ldy, const void *x, int64_t ldx, 
     if (d->algo == RDB_ALGO_AUTO && d->coef_rows == 0) {
         // vector-coef, up to a few thousand tokens, with room for the partial outputs: W tiles spread over all compute units
         rc = linear_fwd_vecsplit(y, ldy, x, ldx, coef, scale_bias, bias, d, num_compute_units(), workspace, workspace_bytes, s);
+        if (rc != RDB_E_UNSUPPORTED) return rc;
+    }
+    if (d->algo == RDB_ALGO_AUTO) {   // a handful of tokens: spread over the chip, at latency
+        rc = linear_fwd_few(y, ldy, x, ldx, coef, scale_bias, bias, d, workspace, workspace_bytes, s);
         if (rc != RDB_E_UNSUPPORTED) return rc;
     }
     if (d->algo == RDB_ALGO_AUTO && d->act_dtype == RDB_BF16 && d->tokens <= 96) {
@@ -1308,9 +1317,10 @@ extern "C" int rdb_linear_bwd_kept(void *dx, int64_t lddx, void *dcoef, int dcoe
     return rc;
 }
 
-// rdb_factored.hip, rdb_smallk.hip
+// rdb_factored.hip, rdb_few.hip, rdb_smallk.hip
 namespace rdb {
 int selftest_giveup_factored(void *y, int64_t ldy, void *state, const void *coef, const rdb_linear_desc *d, int num_cus, int polls, hipStream_t s);
+int selftest_giveup_few(void *y, int64_t ldy, const void *coef, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, int polls, hipStream_t s);
 int selftest_giveup_smallk(void *y, int64_t ldy, const void *coef, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, int polls,
                            hipStream_t s);
 }
@@ -1328,7 +1338,8 @@ extern "C" int rdb_selftest_sync_giveup(void *y, int64_t ldy, void *scratch, int
         if (pl.nchunks != 1 || scratch_bytes < pl.state_stride) rc = RDB_E_UNSUPPORTED;
         else rc = selftest_giveup_factored(y, ldy, scratch, coef, d, num_compute_units(), polls, (hipStream_t)stream);
     } else {
-        rc = selftest_giveup_smallk(y, ldy, coef, d, scratch, scratch_bytes, polls, (hipStream_t)stream);
+        rc = selftest_giveup_few(y, ldy, coef, d, scratch, scratch_bytes, polls, (hipStream_t)stream);
+        if (rc == RDB_E_UNSUPPORTED) rc = selftest_giveup_smallk(y, ldy, coef, d, scratch, scratch_bytes, polls, (hipStream_t)stream);
     }
     if (rc == RDB_E_UNSUPPORTED)
         return set_error(RDB_E_UNSUPPORTED, "rdb_selftest_sync_giveup: needs a layer whose forward has a one-launch form (bf16 matrix-coef, k <= 256, "

@@ -140,7 +140,7 @@ def test_unaligned_views(hip, oracle):
 @pytest.mark.parametrize("in_f,out_f,k", [(1, 2, 3), (2, 9, 1), (3, 5, 2), (4, 6, 5), (5, 3, 7), (17, 15, 18), (66, 131, 19), (129, 65, 33), (259, 126, 65)])
 def test_rows_that_end_inside_a_piece_of_four(hip, oracle, in_f, out_f, k, dtype):
     """Extents of which 1, 2, 3 or all 4 values of a row's last piece exist, and rows of fewer than four values, with NaNs behind every row.
-    Every product accumulates in fp32 (1e-5); what is stored as bf16 is rounded once (2^-9)."""
+    Every product accumulates in fp32 (1e-5); what is stored as bf16 is rounded once (at most 2^-8 of a value)."""
     from randumb_amd._lib import RDB_ALGO_AUTO, RDB_ALGO_FACTORED
 
     algo = RDB_ALGO_FACTORED if dtype == torch.float32 else RDB_ALGO_AUTO   # the factored form of bf16 is that of whole multiples of 8
@@ -153,7 +153,7 @@ def test_rows_that_end_inside_a_piece_of_four(hip, oracle, in_f, out_f, k, dtype
     xs, dys, cc = behind_nans(x), behind_nans(dy), coef.cuda()
     want_y = oracle.linear_fwd(x.float().numpy(), coef.float().numpy(), in_f, out_f, seed)
     want_dx, want_dc, _ = oracle.linear_bwd(x.float().numpy(), dy.float().numpy(), coef.float().numpy(), in_f, out_f, seed)
-    tol = F32_TOL if dtype == torch.float32 else 2.0**-9
+    tol = F32_TOL if dtype == torch.float32 else 2.0**-8
     print(f"case f32 matrix cores edges in={in_f} out={out_f} k={k} {dtype}", flush=True)
     y = hip.linear_fwd(xs, cc, in_f, out_f, in_f, 1, seed, algo=algo)
     assert rel_l2(y.float().cpu().numpy(), want_y) < tol

@@ -1,0 +1,110 @@
+"""Forward pass for a handful of tokens (rdb_few.hip) against float64: sizes around its tiles (16 tokens, 16 coefficients, chunks of 128
+and more input features, 64 output features), odd ones, any alignment, infinities; one launch against two; replays; a wait that gives up."""
+import ctypes
+
+import pytest
+import torch
+
+from randumb_amd import _lib, hip, ops
+
+pytestmark = pytest.mark.gpu
+
+# fp32: sums of up to some thousand products, each rounded at 2^-24 of a running sum; bf16: the same, then rounded once (8 bits: 2^-8 of a value at most)
+TOL = {torch.float32: 2e-6, torch.bfloat16: 2.0**-8}
+
+
+def _case(T, in_f, out_f, k, dtype, seed=5):
+    g = torch.Generator().manual_seed(T * 1000 + k)
+    x, c, b = torch.randn(T, in_f, generator=g), torch.randn(out_f, k, generator=g) / k ** 0.5, torch.randn(out_f, generator=g)
+    return [t.to(dtype).cuda() for t in (x, c, b)] + [ops.sq5_gen_2d(in_f, k, seed).double()]
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,in_f,out_f,k", [(1, 1, 1, 1), (2, 7, 3, 5), (15, 127, 63, 15), (16, 128, 64, 16), (17, 129, 65, 17), (1, 4104, 2049, 16), (32, 513, 257, 128),
+                                            (31, 2056, 2120, 100), (16, 1000, 4100, 129), (13, 4096, 1000, 256), (1, 1030, 70, 257), (32, 1040, 2200, 512),
+                                            (33, 300, 100, 33), (48, 264, 2112, 64), (48, 4100, 300, 250), (47, 1200, 520, 510)])
+def test_against_float64(T, in_f, out_f, k, dtype):
+    print(f"case few T={T} in={in_f} out={out_f} k={k} {dtype}", flush=True)
+    x, c, b, N = _case(T, in_f, out_f, k, dtype)
+    want = (x.double() @ N) @ c.double().t()
+    y = hip.linear_fwd(x, c, in_f, out_f, in_f, 1, 5, bias=b)
+    assert _rel(y, want + b.double()) < TOL[dtype]
+    before = hip.set_one_launch(0)
+    try:
+        assert torch.equal(y, hip.linear_fwd(x, c, in_f, out_f, in_f, 1, 5, bias=b))   # the same sums in the same order
+    finally:
+        hip.set_one_launch(before)
+    # rows that begin anywhere, NaNs around them, y in a wider matrix
+    wide = torch.full((T, in_f + 3), float("nan"), device="cuda", dtype=dtype)
+    wide[:, 1:1 + in_f] = x
+    assert torch.equal(y, hip.linear_fwd(wide[:, 1:1 + in_f], c, in_f, out_f, in_f, 1, 5, bias=b))
+    d = hip._desc(T, in_f, out_f, c, in_f, 1, 5, dtype, 0)
+    need = _lib.load().rdb_linear_workspace_bytes(0, ctypes.byref(d))
+    ws, out = torch.randint(0, 256, (need,), dtype=torch.uint8, device="cuda"), torch.full((T, out_f + 5), 7.0, device="cuda", dtype=dtype)
+    assert _lib.load().rdb_linear_fwd(out.data_ptr(), out_f + 5, x.data_ptr(), in_f, c.data_ptr(), None, b.data_ptr(), ctypes.byref(d), ws.data_ptr(), need,
+                                      torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(out[:, :out_f], y) and bool((out[:, out_f:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [1, 2, 40])
+def test_not_finite(k, dtype):
+    """Infinities and NaNs come out where and as 64-bit arithmetic has them, and nowhere else; very large values stay finite."""
+    T, in_f, out_f = 6, 200, 70
+    x, c, _, N = _case(T, in_f, out_f, k, dtype)
+    inf = float("inf")
+    x[1, 3], x[2, 150], x[3, 7] = inf, -inf, float("nan")
+    x[4] = 0.0
+    x[4, 60] = 1.0e37
+    c[5, 0], c[6, k - 1] = inf, -inf
+    want = (x.double() @ N) @ c.double().t()
+    y = hip.linear_fwd(x, c, in_f, out_f, in_f, 1, 5).double()
+    assert torch.equal(torch.isnan(y), torch.isnan(want))
+    assert torch.equal(torch.isinf(y), torch.isinf(want)) and torch.equal(y[torch.isinf(y)], want[torch.isinf(want)])
+    # against the sum of the terms' sizes: fp32 roundings along the way, and 2^-21 where a sum beside one that is not finite is done again
+    size = (x.double().abs() @ N.abs()) @ c.double().abs().t()
+    bound = 2.0**-19 * size + (0.0 if dtype == torch.float32 else 2.0**-8) * want.abs()
+    ok = torch.isfinite(want)
+    assert bool(((y - want).abs() <= bound)[ok].all())
+
+
+def test_recorded_launches():
+    """Both forms recorded into one graph and replayed on changing inputs, with eager calls in between."""
+    shapes = [(5, 1001, 999, 99), (16, 4096, 4096, 256), (40, 4096, 512, 256)]   # one launch, two, three
+    cases = [_case(*s, torch.bfloat16)[:2] for s in shapes]
+    call = lambda: [hip.linear_fwd(x, c, s[1], s[2], s[1], 1, 5) for s, (x, c) in zip(shapes, cases)]
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for i in range(4):
+        for x, _ in cases:
+            x.copy_(torch.randn(x.shape, generator=torch.Generator().manual_seed(i)))
+        graph.replay()
+        got = [o.clone() for o in out]
+        assert all(torch.equal(a, b) for a, b in zip(got, call())), i
+        torch.cuda.synchronize()
+
+
+# 20 tokens: these kernels; 64: the vector-ALU kernels of rdb_smallk.hip, whose wait is their own
+@pytest.mark.parametrize("T", [20, 64])
+def test_a_wait_that_gives_up(T):
+    """NaN throughout, the counter, and the host's watch, as for the other one-launch forms."""
+    in_f, out_f, k = 1000, 520, 16
+    x, c, _, _ = _case(T, in_f, out_f, k, torch.float32)
+    want = hip.linear_fwd(x, c, in_f, out_f, in_f, 1, 5)
+    d = hip._desc(T, in_f, out_f, c, in_f, 1, 5, torch.float32, 0)
+    ws = torch.zeros(int(_lib.load().rdb_linear_workspace_bytes(0, ctypes.byref(d))), dtype=torch.uint8, device="cuda")
+    y = torch.zeros(T, out_f, device="cuda")
+    hip.selftest_sync_giveup(y, ws, c, in_f, 5, polls=32)
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(y).all())
+    with pytest.raises(_lib.RandumbHipError, match="gave up"):
+        hip.sync_check()
+    hip.set_one_launch(1)
+    assert torch.equal(hip.linear_fwd(x, c, in_f, out_f, in_f, 1, 5), want)

@@ -94,7 +94,7 @@ def test_both_products_over_dy_in_one_launch(T, in_f, out_f, k, dtype):
     y = ops.linear(leaves[0], leaves[1], in_f, out_f, in_f, 1, 8, None, None)
     dx, dc = torch.autograd.grad(y, leaves, dy.cuda(), retain_graph=True)
     D = dy.double()
-    tol = 5e-6 if dtype == torch.float32 else 2.0**-9   # fp32 sums throughout; bf16 results are rounded once
+    tol = 5e-6 if dtype == torch.float32 else 2.0**-8   # fp32 sums throughout; bf16 results are rounded once, by at most 2^-8 of a value
     assert _rel(dx, (D @ c.double()) @ N.t()) < tol and _rel(dc, D.t() @ (x.double() @ N)) < tol
     again = torch.autograd.grad(y, leaves, dy.cuda(), retain_graph=True)
     assert torch.equal(dx, again[0]) and torch.equal(dc, again[1])

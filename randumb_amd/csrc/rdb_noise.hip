@@ -51,6 +51,13 @@ __global__ __launch_bounds__(NT) void sq5_fill_1d_kernel(float *__restrict__ out
 // Thash/s; this form: 3.0 at 768 x 3072 elements, k = 256, 222 -> 200 us, 3.1 at k = 1024).  Also measured: the terms as bytes of an 8-bit
 // matrix operand, without conversion and multiplication on the vector ALU (v_mfma_i32_16x16x64_i8): 229 us.
 constexpr int COEF_CHUNK = 2048;
+// Coefficients below this in magnitude: 2^31 times their terms stays finite, and so do sums of them; others (and NaNs) get the factor 2^-31
+// term by term.  Without it, and with MAT_UNROLL terms a turn of the loop (still one after the other), a term takes 17 vector instructions
+// instead of 19: 768 x 3072 elements, k = 256: 219 -> 205 us, and the pass of that layer, 1024 tokens, 538 -> 520; 4096 rows of a 50304 x
+// 768 table, forward and backward, 525 -> 522 (one term a turn: 540).  The round constants stay literals: in scalar or vector registers the
+// same instructions take 2 to 6 % longer.
+constexpr float MAT_LARGE = 3.777893186295716e22f;   // 2^75
+constexpr int MAT_UNROLL = 8;
 
 struct MatVecParams {
     float *out;
@@ -66,7 +73,7 @@ struct MatVecParams {
 // 4 us).
 template <bool GATHER, int LANES> __global__ __launch_bounds__(NT) void materialize_vec_kernel(MatVecParams p)
 {
-    __shared__ float cs[COEF_CHUNK];
+    __shared__ __align__(16) float cs[COEF_CHUNK];
     const int64_t n = ((int64_t)blockIdx.x * NT + threadIdx.x) / LANES;
     const int part = threadIdx.x % LANES;
     const bool live = n < p.Nw;
@@ -77,16 +84,45 @@ template <bool GATHER, int LANES> __global__ __launch_bounds__(NT) void material
     }
     uint32_t first = a * PN1 + p.seed + (uint32_t)part * SQ5_N1;  // first-round value for m = part; +N1 per step of m
     float acc = 0.0f;
+    int large = 0;   // stays so for the chunks that follow: the sum is large then
     for (int64_t m0 = 0; m0 < p.k; m0 += COEF_CHUNK) {   // a multiple of LANES
         const int cnt = (int)((p.k - m0) < COEF_CHUNK ? (p.k - m0) : COEF_CHUNK);
         __syncthreads();
-        for (int j = threadIdx.x; j < cnt; j += NT) cs[j] = load_as_f32(p.coef, p.coef_dtype, m0 + j);
-        __syncthreads();
+        for (int j = threadIdx.x; j < cnt; j += NT) {
+            const float c = load_as_f32(p.coef, p.coef_dtype, m0 + j);
+            cs[j] = c;
+            large |= !(fabsf(c) < MAT_LARGE);
+        }
+        if (__syncthreads_or(large)) {
+            if (live)
+                for (int j = part; j < cnt; j += LANES) {
+                    acc = fmaf(sq5_unit(sq5_tail_apart(first)), cs[j], acc);
+                    first += LANES * SQ5_N1;
+                }
+            continue;
+        }
         if (live) {
-            for (int j = part; j < cnt; j += LANES) {
-                acc = fmaf(sq5_unit(sq5_tail_apart(first)), cs[j], acc);
+            // 2^31 times the sum: the terms' common factor is taken out of the loop (a power of two: the same roundings)
+            float sum = acc * 2147483648.0f;
+            int j = part;
+            if (LANES == 1) {
+                for (; j + MAT_UNROLL <= cnt; j += MAT_UNROLL) {
+                    float c[MAT_UNROLL];
+#pragma unroll
+                    for (int e = 0; e < MAT_UNROLL; ++e) c[e] = cs[j + e];
+#pragma unroll
+                    for (int e = 0; e < MAT_UNROLL; ++e) {
+                        sum = fmaf((float)(int32_t)sq5_tail_apart(first), c[e], sum);
+                        first += SQ5_N1;
+                        __builtin_amdgcn_sched_barrier(0);   // one term after the other
+                    }
+                }
+            }
+            for (; j < cnt; j += LANES) {
+                sum = fmaf((float)(int32_t)sq5_tail_apart(first), cs[j], sum);
                 first += LANES * SQ5_N1;
             }
+            acc = sum * 4.656612873077392578125e-10f;
         }
     }
 #pragma unroll

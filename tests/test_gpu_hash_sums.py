@@ -86,3 +86,26 @@ def _noise_rows(hip, row, dim, k, seed):
     PRIME, N1, M = 198491317, 0xD2A80A3F, 1 << 32
     # noise(PRIME * (row * dim + r) + m, seed) = the 2-D fill's element (r, m) with the first row's offset folded into the seed
     return hip.sq5_fill_2d(dim, k, (seed + PRIME * row * dim * N1) % M)
+
+
+@pytest.mark.parametrize("n,k", [(1, 1), (3000, 7), (3000, 8), (70001, 9), (300, 2047), (70001, 2049), (300, 2063), (5000, 4100)])
+def test_terms_with_and_without_their_common_factor(hip, n, k):
+    """Coefficients from which on the factor 2^-31 is applied term by term, everywhere or first from the second chunk of 2048 on, or only in the
+    first: powers of two of the same coefficients give the same bits, larger by that power (n: a lane an element, or several)."""
+    print(f"case common factor n={n} k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    c = torch.randn(k, generator=g, device="cuda")
+    values = lambda coef: hip.materialize_fwd(coef, (n,), (1,), 11, None, False)
+    want = values(c)
+    for p in (70, 76, 100):
+        assert torch.equal(values(c * 2.0**p), want * 2.0**p), p
+    for at in sorted({0, k // 2, k - 1}):   # one large coefficient among others
+        big = c * 2.0**-40
+        big[at] = 3.0e37
+        noise = hip.sq5_fill_2d(n, k, 11).double()[:, at] if n <= 5000 else None
+        got = values(big)
+        assert bool(torch.isfinite(got).all())
+        if noise is not None:
+            assert rel(got, noise * 3.0e37) < 1e-6
+    c[k - 1] = float("inf")
+    assert not bool(torch.isfinite(values(c)).any())

@@ -379,7 +379,7 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false, int ES = 4> struct Fg
 // Results leave with streaming stores: they would be written back from L2 at the end of the kernel otherwise, after the last
 // block (y of that layer, 25 MB: 26.4 -> 24.8 us).  Not so where rows are not whole lines of 128 bytes: a streaming store of part of
 // a line goes to memory as such, where L2 puts a line's parts together (y of 3899 tokens x 5603, k = 199: 107 -> 75 us; 1500 x 5245, k =
-// 156: 36 -> 24.6; 4096 x 999, k = 100: 16.7 -> 12.1; on the tiles of rdb_big.hpp in bf16 6000 x 512 -> 6008, k = 320: 61.7 -> 57.0).
+// 156: 36 -> 24.6; 4096 x 999, k = 100: 16.7 -> 15.3; on the tiles of rdb_big.hpp in bf16 6000 x 512 -> 6008, k = 320: 61.7 -> 59.5).
 // AES, BES: bytes per element of the two matrices (SPLIT: 4, or 2, bf16; otherwise 0, see FgOperand).
 // f32_gemm_block: what block (bx, by, bz) of a product does (gx: how many there are along x).  `lds`: FgBlock::LDS floats; not_finite: a
 // word of LDS.
@@ -577,12 +577,16 @@ __device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, 
     const float scale = (EPI != FG_ADD_SCALED && EPI != FG_STORE_RBIAS) ? 0.0f
                         : p.scale_bf16 ? bf16_to_f32(reinterpret_cast<const bf16_t *>(p.scale)[0]) : p.scale[0];
     float dot = 0.0f;
-    auto results = [&](auto stream) __attribute__((always_inline)) {
+    // KIND: how the results leave, where that is known outside of the loops (a branch per store costs 4 us of the fp32 step above)
+    enum { STREAM, PLAIN, NARROW, ANY };
+    auto results = [&](auto kind) __attribute__((always_inline)) {
+        constexpr int KIND = decltype(kind)::value;
+        const bool to16 = KIND == NARROW || (KIND == ANY && o16);
 #pragma unroll
         for (int ni = 0; ni < NI; ++ni) {
             const int n = n0 + wn * 64 + ni * 32 + r;
             if (n >= p.N) continue;
-            const float bv = EPI != FG_STORE_BIAS ? 0.0f : o16 ? bf16_to_f32(reinterpret_cast<const bf16_t *>(p.bias)[n]) : p.bias[n];
+            const float bv = EPI != FG_STORE_BIAS ? 0.0f : to16 ? bf16_to_f32(reinterpret_cast<const bf16_t *>(p.bias)[n]) : p.bias[n];
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
@@ -593,24 +597,25 @@ __device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, 
                     const float a = acc[mi][ni][j];
                     if (EPI == FG_DOT || (EPI == FG_ADD_SCALED && p.dotm)) {
                         const int64_t e = (int64_t)m * p.lddot + n;
-                        dot = fmaf(a, o16 ? bf16_to_f32(reinterpret_cast<const bf16_t *>(p.dotm)[e]) : p.dotm[e], dot);
+                        dot = fmaf(a, to16 ? bf16_to_f32(reinterpret_cast<const bf16_t *>(p.dotm)[e]) : p.dotm[e], dot);
                     }
                     if (EPI != FG_DOT) {
                         const int64_t e = (int64_t)m * p.ldo + n;
                         if (EPI == FG_STORE_RBIAS) out[e] = fmaf(scale, noise1d((uint32_t)m * p.nsR + (uint32_t)n * p.nsK, p.seed), a);
-                        else if (o16) out16[e] = f32_to_bf16(EPI == FG_ADD_SCALED ? fmaf(scale, a, bf16_to_f32(out16[e])) : a + bv);
+                        else if (to16) out16[e] = f32_to_bf16(EPI == FG_ADD_SCALED ? fmaf(scale, a, bf16_to_f32(out16[e])) : a + bv);
                         else if (EPI == FG_ADD_SCALED) out[e] = fmaf(scale, a, out[e]);
-                        else if (decltype(stream)::value) __builtin_nontemporal_store(a + bv, out + e);
+                        else if (KIND == STREAM) __builtin_nontemporal_store(a + bv, out + e);
                         else out[e] = a + bv;
                     }
                 }
         }
     };
     if constexpr (EPI == FG_STORE || EPI == FG_STORE_BIAS) {
-        if (p.ldo % 32 == 0) results(std::true_type{});   // rows of whole lines
-        else results(std::false_type{});
+        if (o16) results(std::integral_constant<int, NARROW>{});
+        else if (p.ldo % 32 == 0) results(std::integral_constant<int, STREAM>{});   // rows of whole lines
+        else results(std::integral_constant<int, PLAIN>{});
     } else {
-        results(std::false_type{});
+        results(std::integral_constant<int, ANY>{});
     }
     if (EPI == FG_DOT || (EPI == FG_ADD_SCALED && p.dotm)) {
         // lanes, then waves, in a fixed order

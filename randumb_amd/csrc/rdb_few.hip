@@ -1,14 +1,17 @@
-// Forward pass of a matrix-coef layer for a handful of tokens (a served model generating): z = x . N^T, y = z . C^T (+ bias) on the
-// matrix cores with 16 x 16 tiles, at fp32 accuracy whatever the operands' type, in one launch.
+// Forward pass of a matrix-coef layer for few tokens (a served model generating, short prompts): z = x . N^T, y = z . C^T (+ bias) on
+// the matrix cores with 16 x 16 tiles, at fp32 accuracy whatever the operands' type, in one to three launches.
 //
 // What bounds it is latency: 16 tokens x 4096 -> 11008, k = 256 move 6 MB and multiply next to nothing.  Contracting blocks (16 coefficients
-// x a chunk of in_f, the tokens all at once, so that every noise value is hashed once) leave partial sums of z; expanding blocks (64
-// output features) have their rows of C in registers by the time these are there, add them up in chunk order, and multiply.  In
-// one launch the contracting blocks come first and publish a tag each (rdb_common.hpp); where the partial sums are so many that
-// reading them around the dies' L2 caches costs more than a launch, the two kinds of block are two launches of the same kernel.
+// x a chunk of in_f x up to 32 tokens, each noise value hashed once for all of them) leave partial sums of z; expanding blocks (64
+// output features x 16 tokens, or 32 where there are more blocks than the chip runs at once) have their rows of C in registers by
+// the time these are there, add them up in chunk order, and multiply.  In one launch the contracting blocks come first and publish
+// a tag each (rdb_common.hpp); where the partial sums are so many that reading them around the dies' L2 caches costs more than a
+// launch, the two kinds of block are two launches of the same kernel.
 // us per call, three launches on the vector ALU (or the kernels for many tokens) -> here: 16 tokens x 4096 -> 11008, k = 256, bf16 14.5 ->
 // 11.5; 1 x 7512 -> 2376, k = 512, bf16 34.6 -> 14.0; 5 x 1001 -> 999, k = 99, bf16 17.1 -> 7.5; 22 x 264 -> 352, k = 64, fp32 17.7 -> 8.6;
-// 1 x 4096 -> 4096, k = 16, fp32 9.0 -> 8.6.  What is left is launches and memory round trips: x in, partial sums out and in, y out.
+// 1 x 4096 -> 4096, k = 16, fp32 9.0 -> 8.6; 64 x 4096 -> 11008, k = 256, bf16 29.2 -> 17.9; 128 x 8192 -> 1024, k = 128, bf16 28.0 -> 15.2;
+// 256 x 512 -> 512, k = 128, fp32 17.4 -> 9.8.  What is left is launches and memory round trips: x in, partial sums out and in, y out.
+// Tokens split finer than they were (48 to a block of either kind): 48 x 768 -> 3072, k = 256, bf16 15.5 -> 10.7, 32 tokens 13.6 -> 10.6.
 //
 // fp32 accuracy: a noise value is exactly three bf16 parts, so its products with bf16 activations are exact in three matrix instructions;
 // so are those of z (fp32) with bf16 coefficients.  fp32 activations and coefficients are split as well: the six largest of the nine
@@ -21,24 +24,27 @@
 
 namespace rdb {
 
-
 constexpr int FEW_ROWS = 64;       // output features of an expanding block: 16 a wave
 constexpr int FEW_COEFS = 16;      // coefficients of a contracting block
 constexpr int FEW_STEPS = 4;       // steps of 32 contraction values a contracting wave hashes ahead of its products
-constexpr int FEW_TOKENS = 48, FEW_K = 512;   // z's three parts in LDS: at most 150 KB
+constexpr int FEW_TOKENS = 256, FEW_K = 512;   // z's three parts of 32 tokens in LDS: at most 100 KB
 
 struct FewParams {
     void *y;
     const void *x, *coef, *bias;
     int64_t ldx, ldy;
-    float *part;   // [chunks][ranges of 16 coefficients][tokens][16]
+    float *part;   // [chunks][tiles of 16 tokens, or fewer if there are no more][ranges of 16 coefficients][tokens of a tile][16]
     int T, in_f, out_f, k, chunks, ranges;
+    int tile, tiles;     // tokens of a tile, tiles
+    int c_groups;        // groups of tokens of the contracting blocks
     int wave_values;     // contraction values per wave and chunk: a multiple of 32
     int x_vec, c_vec, y_vec;   // 16-byte pieces of x and C, 4 values of y at a time
     uint32_t seed;
     int c_blocks;        // contracting blocks of this launch: they come first
+    int e_blocks;        // expanding blocks of a group of tokens
     unsigned long long *slots;   // NULL, or one tag per contracting block
     unsigned long long tag;
+    int tags;
     SyncWait wait;
     unsigned int *count;
     int consumers;
@@ -190,18 +196,25 @@ template <> struct FewSide<float> {
     }
 };
 
-// Block (range, chunk): z[all tokens][16 coefficients] over the chunk, a quarter of it to a wave.
+// Block (range, chunk, group): z[TT tiles of tokens][16 coefficients] over the chunk, a quarter of it to a wave.
 template <typename E, int TT> __device__ __forceinline__ void few_contract(const FewParams &p, int b, float *__restrict__ lds)
 {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
-    const int range = b % p.ranges, ch = b / p.ranges, m = range * FEW_COEFS + r;
+    int range = b % p.ranges, ch = b / p.ranges, group = 0;
+    if (TT > 1) {   // a group's chunk is read by blocks of one die where that comes out even
+        const int pieces = p.chunks * p.c_groups;
+        range = b / pieces;
+        ch = (b - range * pieces) / p.c_groups;
+        group = b - range * pieces - ch * p.c_groups;
+    }
+    const int m = range * FEW_COEFS + r, tile0 = group * TT, t0 = tile0 * 16, T = min(TT * 16, p.T - t0);
     const int i_begin = (ch * 4 + wave) * p.wave_values;
-    const E *const x = static_cast<const E *>(p.x);
+    const E *const x = static_cast<const E *>(p.x) + (int64_t)t0 * p.ldx;
     const E *row[TT];
     bool live[TT];
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
-        live[tt] = tt * 16 + r < p.T;
+        live[tt] = tt * 16 + r < T;
         row[tt] = x + (int64_t)(live[tt] ? tt * 16 + r : 0) * p.ldx;
     }
     f32x4 acc[TT], low[TT];
@@ -228,12 +241,12 @@ template <typename E, int TT> __device__ __forceinline__ void few_contract(const
             }
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt) {
-            if (tt * 16 >= p.T) break;   // uniform
+            if (tt * 16 >= T) break;   // uniform
             FewSide<E> a[FEW_STEPS];
 #pragma unroll
             for (int s = 0; s < FEW_STEPS; ++s)
                 if (i0 + s * 32 < p.wave_values) a[s].set(raw[s]);
-            if (tt + 1 < TT && (tt + 1) * 16 < p.T) request(tt + 1);
+            if (tt + 1 < TT && (tt + 1) * 16 < T) request(tt + 1);
 #pragma unroll
             for (int s = 0; s < FEW_STEPS; ++s)
                 if (i0 + s * 32 < p.wave_values) a[s].mma_a(acc[tt], low[tt], noise[s]);
@@ -245,28 +258,28 @@ template <typename E, int TT> __device__ __forceinline__ void few_contract(const
 #pragma unroll
         for (int j = 0; j < 4; ++j) lds[((wave * TT + tt) * 16 + g * 4 + j) * 16 + r] = acc[tt][j] + low[tt][j];
     __syncthreads();
-    float *const out = p.part + (int64_t)(ch * p.ranges + range) * p.T * 16;
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
         const int t = tt * 16 + (tid >> 4);
-        if (t < p.T) {
+        if (t < T) {
+            float *const out = p.part + (((int64_t)ch * p.tiles + tile0 + tt) * p.ranges + range) * p.tile * 16;
             float v = lds[tt * 256 + tid];
 #pragma unroll
             for (int w = 1; w < 4; ++w) v += lds[(w * TT + tt) * 256 + tid];
-            __hip_atomic_store(out + (int64_t)t * 16 + (tid & 15), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(out + tid, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }
 
-// Block: 64 output features, all tokens.
-template <typename E, int KS, int TT> __device__ __forceinline__ void few_expand(const FewParams &p, int b, unsigned char *__restrict__ smem)
+// Block: 64 output features, TT tiles of tokens.  MANY: tiles have 16 tokens
+template <typename E, int KS, int TT, bool MANY> __device__ __forceinline__ void few_expand(const FewParams &p, int b, unsigned char *__restrict__ smem)
 {
     constexpr int KW = KS * 32, LD = KW + 8;   // 16 bytes of padding: 16 rows' pieces lie in different banks
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
-    const int o0 = b * FEW_ROWS + wave * 16;
+    const int tile = MANY ? 16 : p.tile, tile0 = MANY ? b / p.e_blocks * TT : 0, t0 = tile0 * 16, T = min(TT * 16, p.T - t0), ob = MANY ? b % p.e_blocks : b, o0 = ob * FEW_ROWS + wave * 16;
     bf16_t *const planes = reinterpret_cast<bf16_t *>(smem);
-    const int PLANE = (p.T + 15) / 16 * 16 * LD;
-    E *const y = static_cast<E *>(p.y);
+    const int PLANE = (T + 15) / 16 * 16 * LD;
+    E *const y = static_cast<E *>(p.y) + (int64_t)t0 * p.ldy;
     // the wave's rows of C, before anything is waited for
     FewRaw<E> c[KS];
     {
@@ -277,7 +290,7 @@ template <typename E, int KS, int TT> __device__ __forceinline__ void few_expand
     }
     if (p.slots) {
         __shared__ int verdict;
-        const int n = p.chunks * p.ranges;
+        const int n = p.tags;
         if (tid < 64) {
             bool there = false;
             for (int it = 0; it < p.wait.polls && !there; ++it) {
@@ -300,16 +313,16 @@ template <typename E, int KS, int TT> __device__ __forceinline__ void few_expand
         }
         __syncthreads();
         if (verdict == 0) {   // gave up: the block's share of the output becomes NaN, never a sum of whatever is in memory
-            for (int i = tid; i < p.T * FEW_ROWS; i += 256) {
-                const int t = i / FEW_ROWS, o = b * FEW_ROWS + i % FEW_ROWS;
+            for (int i = tid; i < T * FEW_ROWS; i += 256) {
+                const int t = i / FEW_ROWS, o = ob * FEW_ROWS + i % FEW_ROWS;
                 if (o < p.out_f) elem<E>::store(y + (int64_t)t * p.ldy + o, __uint_as_float(0x7fc00000u));
             }
             return;
         }
     }
     // z: four coefficients of a token at a time, the chunks' sums in chunk order, then its three parts
-    const int n4 = p.ranges * p.T * 4;
-    const int64_t stride = (int64_t)p.ranges * p.T * 16;
+    const int per = p.ranges * tile, n4 = min(TT, p.tiles - tile0) * per * 4;
+    const int64_t stride = (int64_t)p.tiles * per * 16, first = (int64_t)tile0 * per * 16;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(p.part, 0, (int)(stride * p.chunks * 4), 0x00020000);
     // IB entries of CB chunks in flight
     auto add_up = [&](auto ib_, auto cb_) __attribute__((always_inline)) {
@@ -322,7 +335,7 @@ template <typename E, int KS, int TT> __device__ __forceinline__ void few_expand
                 for (int i = 0; i < IB; ++i)
 #pragma unroll
                     for (int q = 0; q < CB; ++q) {
-                        const int at = (int)(((int64_t)min(c0 + q, p.chunks - 1) * stride + (int64_t)min(i0 + i * 256, n4 - 1) * 4) * 4);
+                        const int at = (int)(((int64_t)min(c0 + q, p.chunks - 1) * stride + first + (int64_t)min(i0 + i * 256, n4 - 1) * 4) * 4);
                         u[i][q] = __builtin_bit_cast(f32x4, p.slots ? __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, SCOPE_DEVICE) : __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
                     }
 #pragma unroll
@@ -337,7 +350,7 @@ template <typename E, int KS, int TT> __device__ __forceinline__ void few_expand
             for (int i = 0; i < IB; ++i) {
                 const int e = i0 + i * 256;
                 if (e >= n4) continue;
-                const int rt = e >> 2, range = rt / p.T, t = rt - range * p.T, m = range * FEW_COEFS + (e & 3) * 4;
+                const int sub = TT > 1 && (e >> 2) >= per ? 1 : 0, rt = (e >> 2) - sub * per, range = rt / tile, t = sub * 16 + rt - range * tile, m = range * FEW_COEFS + (e & 3) * 4;
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     if (m + j >= p.k) v[i][j] = 0.0f;
@@ -357,9 +370,9 @@ template <typename E, int KS, int TT> __device__ __forceinline__ void few_expand
     // coefficients beyond the last range meet zeros of C: they must be finite
     const int tail4 = (KW - p.ranges * FEW_COEFS) / 4;
     if (tail4 > 0)
-        for (int e = tid; e < 3 * p.T * tail4; e += 256) {
-            const int row = e / tail4, pl = row / p.T;
-            *reinterpret_cast<uint2 *>(planes + pl * PLANE + (row - pl * p.T) * LD + p.ranges * FEW_COEFS + (e - row * tail4) * 4) = make_uint2(0u, 0u);
+        for (int e = tid; e < 3 * T * tail4; e += 256) {
+            const int row = e / tail4, pl = row / T;
+            *reinterpret_cast<uint2 *>(planes + pl * PLANE + (row - pl * T) * LD + p.ranges * FEW_COEFS + (e - row * tail4) * 4) = make_uint2(0u, 0u);
         }
     __syncthreads();
     f32x4 acc[TT], low[TT];
@@ -374,7 +387,7 @@ template <typename E, int KS, int TT> __device__ __forceinline__ void few_expand
             a.template set<ANY>(c[s]);
 #pragma unroll
             for (int tt = 0; tt < TT; ++tt) {
-                if (tt * 16 >= p.T) break;
+                if (tt * 16 >= T) break;
                 const bf16_t *const src = planes + (tt * 16 + r) * LD + s * 32 + g * 8;   // tokens from T on: whatever lies there, in columns nobody stores
                 Split8 z = {*reinterpret_cast<const bf16x8 *>(src), *reinterpret_cast<const bf16x8 *>(src + PLANE), *reinterpret_cast<const bf16x8 *>(src + 2 * PLANE)};
                 if (ANY) z = few_split8_any(few_join8(z));
@@ -387,7 +400,7 @@ template <typename E, int KS, int TT> __device__ __forceinline__ void few_expand
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) zero = tt * 16 + r < p.T ? fmaf(acc[tt][j] + low[tt][j], 0.0f, zero) : zero;
+        for (int j = 0; j < 4; ++j) zero = tt * 16 + r < T ? fmaf(acc[tt][j] + low[tt][j], 0.0f, zero) : zero;
     if (__any(zero != 0.0f)) product(std::true_type{});
     // result element j of lane (r, g): output feature o0 + 4 g + j, token r
     const int o = o0 + g * 4;
@@ -397,7 +410,7 @@ template <typename E, int KS, int TT> __device__ __forceinline__ void few_expand
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
         const int t = tt * 16 + r;
-        if (t >= p.T || o >= p.out_f) continue;
+        if (t >= T || o >= p.out_f) continue;
         float v[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] = acc[tt][j] + low[tt][j] + bv[j];
@@ -431,43 +444,68 @@ __global__ __launch_bounds__(256) void few_sum_kernel(float *__restrict__ part, 
     *at = v;
 }
 
-template <typename E, int KS, int TT> __global__ __launch_bounds__(256, 1) void few_fwd_kernel(FewParams p)
+// TC, TE: tiles of tokens of a contracting and of an expanding block
+template <typename E, int KS, int TC, int TE> __global__ __launch_bounds__(256, 1) void few_fwd_kernel(FewParams p)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const int b = blockIdx.x;
     if (b >= p.c_blocks) {
-        few_expand<E, KS, TT>(p, b - p.c_blocks, smem);
+        few_expand<E, KS, TE, TC == 2>(p, b - p.c_blocks, smem);
         return;
     }
     if (p.slots && threadIdx.x == 0) __hip_atomic_store(p.slots + b, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // a replay may find its tag
-    few_contract<E, TT>(p, b, reinterpret_cast<float *>(smem));
+    few_contract<E, TC>(p, b, reinterpret_cast<float *>(smem));
     if (!p.slots) return;
     if (b == 0 && threadIdx.x == 0) __hip_atomic_store(p.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     publish_tag(p.slots + b, p.tag);
 }
 
 // ----------------------------------------------------------------------------------------------- host side
-// Where these kernels are ahead of those of rdb_smallk.hip, rdb_factored.hip and rdb_f32.hip (us per call, before -> here): bf16 up to 48
-// tokens (40 x 8192 -> 8192, k = 64: 20.5 -> 15.6; 64 x 768 -> 3072, k = 256: 14.6 -> 17.6); fp32, six products instead of three,
-// up to 48 tokens with k <= 64 (48 x 1384 -> 3328, k = 32: 14.2 -> 12.3), 32 with k <= 128 (32 x 2048 -> 2048, k = 128: 13.0 -> 11.2), 16
-// with k <= 256 (24 x 4096 -> 4096, k = 256: 14.6 -> 16.0), and again 32 beyond, where the others have no kernel for few tokens.
+// Where these kernels are ahead of those of rdb_smallk.hip, rdb_factored.hip and rdb_f32.hip.  `units` are the expanding blocks of one
+// tile of tokens: each splits its tokens' z again, so the more of them there are, and the larger k, the sooner the kernels that
+// make z once for wide tiles win; fp32 multiplies twice as much.  us per call, those kernels -> here:
+//   k <= 64    128 x 2048 -> 2048, k = 64: bf16 16.1 -> 9.1, fp32 17.1 -> 10.0; 128 x 3000 -> 11008, k = 64 (1376 units): 18.9 ->
+//              14.1 and 19.6 -> 16.8; 256 x 8192 -> 8192 (2048): fp32 24.4 -> 27.9
+//   k <= 128   128 x 8192 -> 8192: bf16 25.8 -> 18.3, fp32 25.1 -> 22.3 (1024 units); 192 (1536): 29.7 -> 23.1, fp32 26.1 -> 30.0
+//   k <= 256   128 x 4096 -> 4096: bf16 20.9 -> 18.5, fp32 24.6 -> 22.2 (512 units); 160 (640): 22.4 -> 23.0 and 25.6 -> 30.5;
+//              96 x 4096 -> 11008: 39 -> 22.3 and 39.4 -> 32.1; fp32 48 x 5000 -> 600, k = 200: 16.6 -> 19.1
+//   beyond     64 x 1024 -> 4096, k = 512: bf16 17.8 -> 16.0; 64 x 1504 -> 6000, k = 304 (376 units): 17.1 -> 18.5;
+//              fp32 32 x 8192 -> 11008, k = 512: 39 -> 33, 48 tokens 33 -> 50
+// bf16 contractions of at most 512 are short for the kernels of rdb_factored.hip too: 160 x 384 -> 8000, k = 24 (1250 units): 10.7 -> 11.1;
+// 128 x 512 -> 4096, k = 256 (512 units): 12.8 -> 13.1; 64 tokens (256): 12.4 -> 10.1.
+// 256 tokens are the most all the same, though 512 x 768 -> 3072, k = 64 would be 13.4 -> 12.7 (fp32 16.8 -> 15.0): beyond, y stays bit
+// for bit that of the forms that keep z for a backward pass.
 // The factored form is taken as far as everywhere: up to 16 times the products of one with a stored weight.
+static bool few_pays(const rdb_linear_desc *d)
+{
+    const int64_t T = d->tokens, k = d->k, units = cdiv(d->out_f, FEW_ROWS) * cdiv(T, 16);
+    const bool b16 = d->act_dtype == RDB_BF16;
+    if (T <= 16) return true;
+    if (T > FEW_TOKENS) return false;
+    if (b16 && d->in_f <= 512 && units > (k <= 128 ? 512 : 256)) return false;
+    if (k <= 128) return units <= (b16 || k <= 64 ? 1536 : 1024);
+    if (k > 256) return T <= 32 || (b16 && T <= 96 && units <= 300);
+    return b16 ? T <= 96 || units <= 512 : (T <= 96 || (T <= 192 && units <= 512)) && d->in_f <= 4 * d->out_f;
+}
 static bool few_ok(const rdb_linear_desc *d)
 {
     const bool f32 = d->act_dtype == RDB_F32 && d->coef_dtype == RDB_F32, b16 = d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16;
-    const int most = b16 || d->k <= 64 ? FEW_TOKENS : d->k <= 128 || d->k > 256 ? 32 : 16;
-    return (f32 || b16) && d->algo == RDB_ALGO_AUTO && d->coef_rows != 0 && d->k > 0 && d->k <= FEW_K && d->tokens > 0 && d->tokens <= most && d->in_f > 0 &&
-           d->out_f > 0 && d->in_f < (1 << 20) && d->out_f < (1 << 24) && d->k * (d->in_f + d->out_f) < 16 * d->in_f * d->out_f;
+    return (f32 || b16) && d->algo == RDB_ALGO_AUTO && d->coef_rows != 0 && d->k > 0 && d->k <= FEW_K && d->tokens > 0 && d->in_f > 0 &&
+           d->out_f > 0 && d->in_f < (1 << 20) && d->out_f < (1 << 24) && few_pays(d) && d->k * (d->in_f + d->out_f) < 16 * d->in_f * d->out_f;
 }
 // Chunks: about eight of them (sixteen where there is one range of coefficients), of 128 to 512 values (a contracting block hashes a chunk for 16 coefficients: 128 values cost it 0.6 us;
 // an expanding block reads eight at a time: 1 x 4096 -> 4096, k = 16: chunks of 128, 256, 512, 1024: 8.9, 8.0, 8.2, 10.9 us).
-// sum: beyond 200 KB of partial sums they are added up once, by a launch of its own, and not by every expanding block
-// (32 tokens x 4096 -> 11008, k = 256: 15.6 -> 14.9 us; 16 tokens, 131 KB: 11.5, and 12.7 with it).
+// te: tiles of an expanding block.  Finer is sooner ready while the blocks run side by side, two (of k > 128: one) to a compute unit: 64 x
+// 768 -> 3072, k = 64: 8.2 us, two tiles 9.1; 80 x 8192 -> 8192, k = 64, 640 blocks of one tile: 18.7, two tiles 15.1.
+// sum: beyond 200 KB of partial sums for a block they are added up once, by a launch of its own, and not by every expanding block
+// (48 to a block, 32 tokens x 4096 -> 11008, k = 256: 15.6 -> 14.9 us; 16 tokens, 131 KB: 11.5, and 12.7 with it).
 // one: a single launch where the expanding blocks are few and the partial sums small; tags and reads that go around L2 cost many
 // blocks more than a launch does (5 x 1001 -> 999, k = 99: two launches 9.2, one 7.5; 16 x 4096 -> 11008, k = 256: 11.5 and 13.5; 1 x 4096
 // -> 4096, k = 16: 8.0 and 8.6, but a program's host takes 10.7 to issue two).
 struct FewPlan {
     int wave_values, chunks, ranges;
+    int tile, tiles, tc, te;
+    int c_blocks, e_blocks;
     bool sum, one;
     int64_t part_bytes;
 };
@@ -475,16 +513,24 @@ static FewPlan few_plan(const rdb_linear_desc *d)
 {
     FewPlan f;
     f.ranges = (int)cdiv(d->k, FEW_COEFS);
+    f.tile = (int)std::min<int64_t>(d->tokens, 16);
+    f.tiles = (int)cdiv(d->tokens, f.tile);
+    f.tc = f.tiles > 1 ? 2 : 1;
+    const int64_t rows = cdiv(d->out_f, FEW_ROWS), c_groups = cdiv(f.tiles, f.tc);
+    f.te = f.tiles > 1 && rows * f.tiles > (d->k <= 128 ? 512 : 256) ? 2 : 1;
     int64_t chunk = 128;
     while (chunk < 512 && chunk * (f.ranges == 1 ? 16 : 8) < d->in_f) chunk *= 2;
-    const int64_t per_chunk = (int64_t)f.ranges * d->tokens * FEW_COEFS * 4;
-    f.sum = cdiv(d->in_f, chunk) * per_chunk > 200 * 1024;
-    if (f.sum && chunk > 256) chunk = 256;
+    if (c_groups > 1)
+        while ((chunk < 1024 && cdiv(d->in_f, chunk) * f.ranges * c_groups > 512) || cdiv(d->in_f, chunk) > 64) chunk *= 2;   // two blocks a compute unit; the workspace
+    const int64_t per_chunk = (int64_t)f.ranges * f.tile * FEW_COEFS * 4;   // of a tile
+    f.sum = cdiv(d->in_f, chunk) * per_chunk * std::min(f.te, f.tiles) > 200 * 1024;
+    if (f.sum && chunk > 256 && c_groups == 1) chunk = 256;
     f.wave_values = (int)chunk / 4;
     f.chunks = (int)cdiv(d->in_f, chunk);
-    f.part_bytes = f.chunks * per_chunk;
-    const int64_t e_blocks = cdiv(d->out_f, FEW_ROWS);
-    f.one = !f.sum && ((e_blocks <= 32 && f.part_bytes <= 100 * 1024) || (e_blocks <= 80 && f.part_bytes <= 32 * 1024));
+    f.part_bytes = f.chunks * per_chunk * f.tiles;
+    f.c_blocks = (int)(f.chunks * f.ranges * c_groups);
+    f.e_blocks = (int)(rows * cdiv(f.tiles, f.te));
+    f.one = !f.sum && ((f.e_blocks <= 32 && f.part_bytes <= 100 * 1024) || (f.e_blocks <= 80 && f.part_bytes <= 32 * 1024));
     return f;
 }
 
@@ -492,39 +538,38 @@ int64_t linear_few_workspace(const rdb_linear_desc *d)
 {
     if (!few_ok(d)) return 0;
     const FewPlan f = few_plan(d);
-    return f.part_bytes + (int64_t)f.chunks * f.ranges * 8 + 8;   // ... the tags, and the consumers' counter
+    return f.part_bytes + (int64_t)f.c_blocks * 8 + 8;   // ... the tags, and the consumers' counter
 }
 
-template <typename E, int KS, int TT> static int few_launch(FewParams p, int c_blocks, int e_blocks, bool one, bool sum, hipStream_t s)
+template <typename E, int KS, int TC, int TE> static int few_launch(FewParams p, const FewPlan &f, int c_blocks, bool one, hipStream_t s)
 {
-    const size_t smem_z = (size_t)4 * TT * 1024, smem_y = (size_t)3 * cdiv(p.T, 16) * 16 * (KS * 32 + 8) * 2, smem = std::max(smem_z, smem_y);
-    const auto kernel = few_fwd_kernel<E, KS, TT>;
+    const size_t smem_z = (size_t)4 * TC * 1024, smem_y = (size_t)3 * TE * 16 * (KS * 32 + 8) * 2, smem = std::max(smem_z, smem_y);
+    const auto kernel = few_fwd_kernel<E, KS, TC, TE>;
     if (int rc = reserve_lds(reinterpret_cast<const void *>(kernel), smem, "few_fwd_kernel")) return rc;
     p.c_blocks = c_blocks;
     if (one) {
-        kernel<<<(unsigned)(c_blocks + e_blocks), 256, smem, s>>>(p);
+        kernel<<<(unsigned)(c_blocks + f.e_blocks), 256, smem, s>>>(p);
         return check_launch("few_fwd_kernel");
     }
     kernel<<<(unsigned)c_blocks, 256, smem_z, s>>>(p);
     if (int rc = check_launch("few_fwd_kernel (z)")) return rc;
-    if (sum) {
-        const int64_t n4 = (int64_t)p.ranges * p.T * 4;
+    if (f.sum) {
+        const int64_t n4 = (int64_t)p.tiles * p.ranges * p.tile * 4;
         few_sum_kernel<<<(unsigned)cdiv(n4, 256), 256, 0, s>>>(p.part, n4, p.chunks);
         if (int rc = check_launch("few_sum_kernel")) return rc;
         p.chunks = 1;
     }
     p.c_blocks = 0;
-    kernel<<<(unsigned)e_blocks, 256, smem_y, s>>>(p);
+    kernel<<<(unsigned)f.e_blocks, 256, smem_y, s>>>(p);
     return check_launch("few_fwd_kernel (y)");
 }
-template <typename E> static int few_dispatch(const FewParams &p, int c_blocks, int e_blocks, bool one, bool sum, hipStream_t s)
+template <typename E> static int few_dispatch(const FewParams &p, const FewPlan &f, int c_blocks, bool one, hipStream_t s)
 {
-    const int tt = (p.T + 15) / 16;
     auto of = [&](auto ks_) {
         constexpr int KS = decltype(ks_)::value;
-        if (tt == 1) return few_launch<E, KS, 1>(p, c_blocks, e_blocks, one, sum, s);
-        if (tt == 2) return few_launch<E, KS, 2>(p, c_blocks, e_blocks, one, sum, s);
-        return few_launch<E, KS, 3>(p, c_blocks, e_blocks, one, sum, s);
+        if (f.tc == 1) return few_launch<E, KS, 1, 1>(p, f, c_blocks, one, s);
+        if (f.te == 1) return few_launch<E, KS, 2, 1>(p, f, c_blocks, one, s);
+        return few_launch<E, KS, 2, 2>(p, f, c_blocks, one, s);
     };
     if (p.k <= 128) return of(std::integral_constant<int, 4>{});
     if (p.k <= 256) return of(std::integral_constant<int, 8>{});
@@ -549,6 +594,10 @@ static FewParams few_params(const rdb_linear_desc *d, const FewPlan &f, void *y,
     p.k = (int)d->k;
     p.chunks = f.chunks;
     p.ranges = f.ranges;
+    p.tile = f.tile;
+    p.tiles = f.tiles;
+    p.c_groups = (int)cdiv(f.tiles, f.tc);
+    p.e_blocks = (int)cdiv(d->out_f, FEW_ROWS);
     p.wave_values = f.wave_values;
     p.x_vec = d->in_f % 8 == 0 && ldx * es % 16 == 0 && ((uintptr_t)x & 15) == 0;
     p.c_vec = d->k % 8 == 0 && ((uintptr_t)coef & 15) == 0;
@@ -556,13 +605,14 @@ static FewParams few_params(const rdb_linear_desc *d, const FewPlan &f, void *y,
     p.seed = d->seed;
     return p;
 }
-static int few_tags(FewParams &p, const FewPlan &f, int e_blocks, int polls)
+static int few_tags(FewParams &p, const FewPlan &f, int polls)
 {
     p.slots = reinterpret_cast<unsigned long long *>(reinterpret_cast<char *>(p.part) + f.part_bytes);
     p.tag = next_sync_tag();
     p.wait = {nullptr, nullptr, polls};
-    p.count = reinterpret_cast<unsigned int *>(p.slots + (int64_t)f.chunks * f.ranges);
-    p.consumers = e_blocks;
+    p.tags = f.c_blocks;
+    p.count = reinterpret_cast<unsigned int *>(p.slots + f.c_blocks);
+    p.consumers = f.e_blocks;
     return sync_giveups_ptr(&p.wait.giveups);
 }
 
@@ -573,12 +623,11 @@ int linear_fwd_few(void *y, int64_t ldy, const void *x, int64_t ldx, const void 
     if (scale_bias || !few_ok(d) || !workspace || ((uintptr_t)workspace & 15) || workspace_bytes < linear_few_workspace(d)) return RDB_E_UNSUPPORTED;
     const FewPlan f = few_plan(d);
     FewParams p = few_params(d, f, y, ldy, x, ldx, coef, bias, workspace);
-    const int c_blocks = f.chunks * f.ranges, e_blocks = (int)cdiv(d->out_f, FEW_ROWS);
     const bool one = f.one && one_launch_mode();
     if (one) {
-        if (int rc = few_tags(p, f, e_blocks, SYNC_SPIN_LIMIT)) return rc;
+        if (int rc = few_tags(p, f, SYNC_SPIN_LIMIT)) return rc;
     }
-    return d->act_dtype == RDB_BF16 ? few_dispatch<bf16_t>(p, c_blocks, e_blocks, one, f.sum, s) : few_dispatch<float>(p, c_blocks, e_blocks, one, f.sum, s);
+    return d->act_dtype == RDB_BF16 ? few_dispatch<bf16_t>(p, f, f.c_blocks, one, s) : few_dispatch<float>(p, f, f.c_blocks, one, s);
 }
 
 // Test hook: only the expanding blocks of the one-launch form, waiting (at most `polls` polls each) for tags that nobody publishes.
@@ -588,9 +637,8 @@ int selftest_giveup_few(void *y, int64_t ldy, const void *coef, const rdb_linear
     const FewPlan f = few_plan(d);
     if (!f.one) return RDB_E_UNSUPPORTED;
     FewParams p = few_params(d, f, y, ldy, nullptr, 0, coef, nullptr, workspace);
-    const int e_blocks = (int)cdiv(d->out_f, FEW_ROWS);
-    if (int rc = few_tags(p, f, e_blocks, polls)) return rc;
-    return d->act_dtype == RDB_BF16 ? few_dispatch<bf16_t>(p, 0, e_blocks, true, false, s) : few_dispatch<float>(p, 0, e_blocks, true, false, s);
+    if (int rc = few_tags(p, f, polls)) return rc;
+    return d->act_dtype == RDB_BF16 ? few_dispatch<bf16_t>(p, f, 0, true, s) : few_dispatch<float>(p, f, 0, true, s);
 }
 
 }  // namespace rdb

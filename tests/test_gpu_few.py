@@ -1,4 +1,4 @@
-"""Forward pass for a handful of tokens (rdb_few.hip) against float64: sizes around its tiles (16 tokens, 16 coefficients, chunks of 128
+"""Forward pass for few tokens (rdb_few.hip) against float64: sizes around its tiles (16 tokens, 16 coefficients, chunks of 128
 and more input features, 64 output features), odd ones, any alignment, infinities; one launch against two; replays; a wait that gives up."""
 import ctypes
 
@@ -26,7 +26,10 @@ def _rel(a, b):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T,in_f,out_f,k", [(1, 1, 1, 1), (2, 7, 3, 5), (15, 127, 63, 15), (16, 128, 64, 16), (17, 129, 65, 17), (1, 4104, 2049, 16), (32, 513, 257, 128),
                                             (31, 2056, 2120, 100), (16, 1000, 4100, 129), (13, 4096, 1000, 256), (1, 1030, 70, 257), (32, 1040, 2200, 512),
-                                            (33, 300, 100, 33), (48, 264, 2112, 64), (48, 4100, 300, 250), (47, 1200, 520, 510)])
+                                            (33, 300, 100, 33), (48, 264, 2112, 64), (48, 4100, 300, 250), (47, 1200, 520, 510),
+                                            # one tile of tokens and two to an expanding block, the last group not full
+                                            (49, 130, 65, 17), (97, 264, 5100, 40), (96, 260, 2800, 256), (81, 515, 130, 129), (90, 700, 2850, 300),
+                                            (192, 2050, 1000, 131), (256, 1001, 999, 100), (240, 600, 3000, 16), (255, 264, 352, 64)])
 def test_against_float64(T, in_f, out_f, k, dtype):
     print(f"case few T={T} in={in_f} out={out_f} k={k} {dtype}", flush=True)
     x, c, b, N = _case(T, in_f, out_f, k, dtype)
@@ -91,8 +94,8 @@ def test_recorded_launches():
         torch.cuda.synchronize()
 
 
-# 20 tokens: these kernels; 64: the vector-ALU kernels of rdb_smallk.hip, whose wait is their own
-@pytest.mark.parametrize("T", [20, 64])
+# 20 and 64 tokens: these kernels, one group of tokens and several; 264: the vector-ALU kernels of rdb_smallk.hip, whose wait is their own
+@pytest.mark.parametrize("T", [20, 64, 264])
 def test_a_wait_that_gives_up(T):
     """NaN throughout, the counter, and the host's watch, as for the other one-launch forms."""
     in_f, out_f, k = 1000, 520, 16

@@ -15,9 +15,13 @@
 // probabilities are, as they lie in the registers, the right operand of the next product.  (Its contraction runs over kv in
 // another order, 4 g + {0..3, 8..11} of every 16 for lane half g, which the left operand's transposing LDS reads follow.)
 //
-// Measured at 8 sequences x 12 heads x 1024 tokens, us: prep 13.5, forward 29.9, dq 44.6, dk / dv 55.8 (144 in all; the stock
-// operators they replace: attention 81 forward, 267 backward, normalisation and rotation some 450).  13 GFLOP forward and 45
-// backward.  No pipe is full (SQ counters, shares of a compute unit's time): matrix cores 24 to 29 %, vector ALU 42 to 48 % (25 % of the
+// A block owns 128 rows, 32 a wave, or (HALVES) 64, two waves to 32 rows that take the two halves of every tile of the other side and
+// add up at the end.  The longest block is then half as long and there are twice as many, but each stages its tiles for half the
+// rows: for grids that do not keep the compute units busy (at_halves).
+//
+// Measured at 8 sequences x 12 heads x 1024 tokens, us: forward 36.7 (13.5 of them prep), backward 79 (the stock operators they
+// replace: attention 81 forward, 267 backward, normalisation and rotation some 450).  13 GFLOP forward and 45 backward.  No pipe is
+// full (SQ counters, shares of a compute unit's time): matrix cores 24 to 29 %, vector ALU 42 to 48 % (25 % of the
 // forward pass in exponentials, 16 a lane for 16 matrix instructions), LDS 32 to 41 % without bank conflicts; two waves a SIMD and a
 // barrier per 64 rows put them one after the other.  The preparing kernel is the vector ALU's (81 %).
 #include "rdb_gemm.hpp"
@@ -25,7 +29,6 @@
 namespace rdb {
 
 constexpr int HD = 64;              // head dimension
-constexpr int AT_ROWS = 128;        // rows a block owns: 32 a wave
 constexpr int AT_TILE = 64;         // rows of the other side a step takes
 constexpr float AT_SCALE = 0.125f;  // 1 / sqrt(HD)
 constexpr float AT_EXP2 = 0.125f * 1.44269504088896340736f;
@@ -183,6 +186,17 @@ __device__ __forceinline__ void at_pack(bf16x8 (&f)[2], const float (&v)[16])
     }
 }
 __device__ __forceinline__ f32x16 at_mma(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+// one accumulator (32 x 32) of a wave in LDS, for the other wave of its rows
+__device__ __forceinline__ void at_put(float *lds, const f32x16 &v, int lane)
+{
+#pragma unroll
+    for (int j = 0; j < 16; ++j) lds[j * 64 + lane] = v[j];
+}
+__device__ __forceinline__ void at_add(f32x16 &v, const float *lds, int lane)
+{
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] += lds[j * 64 + lane];
+}
 // row (0 .. 31) of accumulator element j in lane half g
 __device__ __forceinline__ int at_row(int j, int g) { return 8 * (j >> 2) + 4 * g + (j & 3); }
 
@@ -195,88 +209,106 @@ struct AttnParams {
     float *delta;            // [B * H][T]
     const float *table;
     bf16_t *dqkv;
-    int T, H, BH, nb;        // nb: blocks of 128 rows per head
+    int T, H, BH, nb;        // nb: blocks per head
     float eps;
 };
 
 // Blocks are numbered with the longest first (causal: a block's work grows with its rows' index, or falls with it for dk / dv),
 // all heads of a block index before the next: with a multiple of 8 heads, a head's blocks all run on the die that holds its k and v in its L2.
+// Every second 256 of them, one for each compute unit, come in the opposite order, eights of them so that the dies stay: a
+// compute unit's first two blocks are a long one and a short one.  us in order -> so: 8 x 12 heads x 1024, forward with preparation
+// 38.3 -> 36.7, backward 83.4 -> 79.0; 7 x 12 x 900: 31.3 -> 31.3, 68.5 -> 64.9.
 __device__ __forceinline__ void at_block(const AttnParams &p, int &bh, int &b, int &h, int &rank)
 {
-    rank = (int)blockIdx.x / p.BH;
-    bh = (int)blockIdx.x - rank * p.BH;
+    const int first = (int)blockIdx.x & ~255, at = (int)blockIdx.x & 255, len = min(256, (int)gridDim.x - first) & ~7;
+    const int x = (first & 256) && at < len ? first + len - 8 - (at & ~7) + (at & 7) : (int)blockIdx.x;
+    rank = x / p.BH;
+    bh = x - rank * p.BH;
     b = bh / p.H;
     h = bh - b * p.H;
 }
 
 // ----------------------------------------------------------------------------------------------- forward
-__global__ __launch_bounds__(256, 3) void attn_fwd_kernel(AttnParams p)
+template <bool HALVES> __global__ __launch_bounds__(256, 3) void attn_fwd_kernel(AttnParams p)
 {
-    __shared__ __align__(16) bf16_t ks_[2][AT_TILE * HD], vs_[2][AT_TILE * HD];
+    __shared__ __align__(16) bf16_t tiles[4][AT_TILE * HD];   // K, K, V, V
+    __shared__ float ls_[4][64];
+    bf16_t *const ks_ = tiles[0], *const vs_ = tiles[2];
+    constexpr int TILE = AT_TILE * HD;
     int bh, b, h, rank;
     at_block(p, bh, b, h, rank);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, g = lane >> 5;
-    const int m0 = (p.nb - 1 - rank) * AT_ROWS, q0 = m0 + wave * 32, T = p.T;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = HALVES ? wave >> 1 : 0, r = lane & 31, g = lane >> 5;
+    constexpr int ROWS = HALVES ? 64 : 128;
+    const int m0 = (p.nb - 1 - rank) * ROWS, q0 = m0 + (HALVES ? wave & 1 : wave) * 32, T = p.T;
     const int64_t ld3 = (int64_t)3 * p.H * HD;
     const TileSource qs(p.q + (int64_t)bh * T * HD, HD, T), kg(p.k + (int64_t)bh * T * HD, HD, T);
     const TileSource vg(p.qkv + (int64_t)b * T * ld3 + (2 * p.H + h) * HD, ld3, T);
     bf16x8 qf[4];
     qs.frags(qf, q0);
-    const int last = (m0 + AT_ROWS < T ? m0 + AT_ROWS : T), nt = (last + AT_TILE - 1) / AT_TILE;
+    const int last = (m0 + ROWS < T ? m0 + ROWS : T), nt = (last + AT_TILE - 1) / AT_TILE;
     f32x4 kr[2], vr[2];
     kg.tile(kr, 0);
     vg.tile(vr, 0);
-    at_store_tile(ks_[0], kr);
-    at_store_tile(vs_[0], vr);
+    at_store_tile(ks_, kr);
+    at_store_tile(vs_, vr);
     __syncthreads();
     f32x16 o[2] = {zero16(), zero16()};
     float l = 0.0f;
     for (int t = 0; t < nt; ++t) {
-        const bf16_t *K = ks_[t & 1], *V = vs_[t & 1];
+        const bf16_t *K = ks_ + (t & 1) * TILE, *V = vs_ + (t & 1) * TILE;
         const bool more = t + 1 < nt;
         const int n0 = t * AT_TILE;
         if (more) {
             kg.tile(kr, n0 + AT_TILE);
             vg.tile(vr, n0 + AT_TILE);
         }
-        if (n0 <= q0 + 31) {
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-                f32x16 s = zero16();
+        for (int i = 0; i < (HALVES ? 1 : 2); ++i) {
+            const int kb = HALVES ? half : i;
+            if (n0 + kb * 32 > q0 + 31) continue;   // past the diagonal
+            f32x16 s = zero16();
 #pragma unroll
-                for (int ks = 0; ks < 4; ++ks) s = at_mma(at_row_frag(K, kb * 32, ks, lane), qf[ks], s);
-                float e[16];
+            for (int ks = 0; ks < 4; ++ks) s = at_mma(at_row_frag(K, kb * 32, ks, lane), qf[ks], s);
+            float e[16];
 #pragma unroll
-                for (int j = 0; j < 16; ++j) e[j] = __builtin_amdgcn_exp2f(s[j] * AT_EXP2);
-                if (n0 + kb * 32 + 31 > q0) {   // reaches past the diagonal
+            for (int j = 0; j < 16; ++j) e[j] = __builtin_amdgcn_exp2f(s[j] * AT_EXP2);
+            if (n0 + kb * 32 + 31 > q0) {   // reaches past the diagonal
 #pragma unroll
-                    for (int j = 0; j < 16; ++j)
-                        if (n0 + kb * 32 + at_row(j, g) > q0 + r) e[j] = 0.0f;
-                }
-#pragma unroll
-                for (int j = 0; j < 16; ++j) l += e[j];
-                bf16x8 f[2];
-                at_pack(f, e);
-#pragma unroll
-                for (int st = 0; st < 2; ++st)
-#pragma unroll
-                    for (int db = 0; db < 2; ++db) o[db] = at_mma(at_col_frag(V, db * 32, kb * 2 + st, lane), f[st], o[db]);
+                for (int j = 0; j < 16; ++j)
+                    if (n0 + kb * 32 + at_row(j, g) > q0 + r) e[j] = 0.0f;
             }
+#pragma unroll
+            for (int j = 0; j < 16; ++j) l += e[j];
+            bf16x8 f[2];
+            at_pack(f, e);
+#pragma unroll
+            for (int st = 0; st < 2; ++st)
+#pragma unroll
+                for (int db = 0; db < 2; ++db) o[db] = at_mma(at_col_frag(V, db * 32, kb * 2 + st, lane), f[st], o[db]);
         }
         if (more) {
-            at_store_tile(ks_[(t + 1) & 1], kr);
-            at_store_tile(vs_[(t + 1) & 1], vr);
+            at_store_tile(ks_ + ((t + 1) & 1) * TILE, kr);
+            at_store_tile(vs_ + ((t + 1) & 1) * TILE, vr);
         }
         __syncthreads();
     }
     l += __shfl_xor(l, 32, 64);
+    if constexpr (HALVES) {   // the two waves of a row: each finishes half of the dimensions
+        float *const acc = reinterpret_cast<float *>(tiles);
+        ls_[wave][lane] = l;
+        at_put(acc + wave * 1024, half ? o[0] : o[1], lane);
+        __syncthreads();
+        l += ls_[wave ^ 2][lane];
+        if (half) o[0] = o[1];
+        at_add(o[0], acc + (wave ^ 2) * 1024, lane);
+    }
     const int row = q0 + r;
     if (row >= T) return;
     const float inv = 1.0f / l;
-    if (g == 0) p.lsum[(int64_t)bh * T + row] = log2f(l);
-    bf16_t *out = p.y + ((int64_t)b * T + row) * p.H * HD + h * HD;
+    if (g == 0 && half == 0) p.lsum[(int64_t)bh * T + row] = log2f(l);
+    bf16_t *out = p.y + ((int64_t)b * T + row) * p.H * HD + h * HD + half * 32;
 #pragma unroll
-    for (int db = 0; db < 2; ++db)
+    for (int db = 0; db < (HALVES ? 1 : 2); ++db)
 #pragma unroll
         for (int jq = 0; jq < 4; ++jq) {
             const u32x2 w = {f32x2_to_bf16x2(o[db][jq * 4] * inv, o[db][jq * 4 + 1] * inv), f32x2_to_bf16x2(o[db][jq * 4 + 2] * inv, o[db][jq * 4 + 3] * inv)};
@@ -334,13 +366,16 @@ __device__ __forceinline__ void at_row_grad(bf16_t *out, const bf16_t *x, const 
         }
 }
 
-__global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(AttnParams p)
+template <bool HALVES> __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(AttnParams p)
 {
-    __shared__ __align__(16) bf16_t ks_[2][AT_TILE * HD], vs_[2][AT_TILE * HD];
+    __shared__ __align__(16) bf16_t tiles[4][AT_TILE * HD];   // K, K, V, V
+    bf16_t *const ks_ = tiles[0], *const vs_ = tiles[2];
+    constexpr int TILE = AT_TILE * HD;
     int bh, b, h, rank;
     at_block(p, bh, b, h, rank);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, g = lane >> 5;
-    const int m0 = (p.nb - 1 - rank) * AT_ROWS, q0 = m0 + wave * 32, T = p.T;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = HALVES ? wave >> 1 : 0, r = lane & 31, g = lane >> 5;
+    constexpr int ROWS = HALVES ? 64 : 128;
+    const int m0 = (p.nb - 1 - rank) * ROWS, q0 = m0 + (HALVES ? wave & 1 : wave) * 32, T = p.T;
     const int64_t ld3 = (int64_t)3 * p.H * HD, ld1 = (int64_t)p.H * HD;
     const TileSource qs(p.q + (int64_t)bh * T * HD, HD, T), kg(p.k + (int64_t)bh * T * HD, HD, T);
     const TileSource vg(p.qkv + (int64_t)b * T * ld3 + (2 * p.H + h) * HD, ld3, T);
@@ -364,68 +399,82 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(AttnParams p)
     }
     const int row = q0 + r;
     const float l2 = row < T ? p.lsum[(int64_t)bh * T + row] : 0.0f;
-    if (g == 0 && row < T) p.delta[(int64_t)bh * T + row] = delta;
-    const int last = (m0 + AT_ROWS < T ? m0 + AT_ROWS : T), nt = (last + AT_TILE - 1) / AT_TILE;
+    if (g == 0 && half == 0 && row < T) p.delta[(int64_t)bh * T + row] = delta;
+    const int last = (m0 + ROWS < T ? m0 + ROWS : T), nt = (last + AT_TILE - 1) / AT_TILE;
     f32x4 kr[2], vr[2];
     kg.tile(kr, 0);
     vg.tile(vr, 0);
-    at_store_tile(ks_[0], kr);
-    at_store_tile(vs_[0], vr);
+    at_store_tile(ks_, kr);
+    at_store_tile(vs_, vr);
     __syncthreads();
     f32x16 dq[2] = {zero16(), zero16()};
     for (int t = 0; t < nt; ++t) {
-        const bf16_t *K = ks_[t & 1], *V = vs_[t & 1];
+        const bf16_t *K = ks_ + (t & 1) * TILE, *V = vs_ + (t & 1) * TILE;
         const bool more = t + 1 < nt;
         const int n0 = t * AT_TILE;
         if (more) {
             kg.tile(kr, n0 + AT_TILE);
             vg.tile(vr, n0 + AT_TILE);
         }
-        if (n0 <= q0 + 31) {
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-                f32x16 s = zero16(), d = zero16();
+        for (int i = 0; i < (HALVES ? 1 : 2); ++i) {
+            const int kb = HALVES ? half : i;
+            if (n0 + kb * 32 > q0 + 31) continue;   // past the diagonal
+            f32x16 s = zero16(), d = zero16();
 #pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-                    s = at_mma(at_row_frag(K, kb * 32, ks, lane), qf[ks], s);
-                    d = at_mma(at_row_frag(V, kb * 32, ks, lane), df[ks], d);
-                }
-                float e[16];
-#pragma unroll
-                for (int j = 0; j < 16; ++j) e[j] = __builtin_amdgcn_exp2f(fmaf(s[j], AT_EXP2, -l2));
-                if (n0 + kb * 32 + 31 > q0) {
-#pragma unroll
-                    for (int j = 0; j < 16; ++j)
-                        if (n0 + kb * 32 + at_row(j, g) > q0 + r) e[j] = 0.0f;
-                }
-#pragma unroll
-                for (int j = 0; j < 16; ++j) e[j] *= d[j] - delta;
-                bf16x8 f[2];
-                at_pack(f, e);
-#pragma unroll
-                for (int st = 0; st < 2; ++st)
-#pragma unroll
-                    for (int db = 0; db < 2; ++db) dq[db] = at_mma(at_col_frag(K, db * 32, kb * 2 + st, lane), f[st], dq[db]);
+            for (int ks = 0; ks < 4; ++ks) {
+                s = at_mma(at_row_frag(K, kb * 32, ks, lane), qf[ks], s);
+                d = at_mma(at_row_frag(V, kb * 32, ks, lane), df[ks], d);
             }
+            float e[16];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) e[j] = __builtin_amdgcn_exp2f(fmaf(s[j], AT_EXP2, -l2));
+            if (n0 + kb * 32 + 31 > q0) {
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    if (n0 + kb * 32 + at_row(j, g) > q0 + r) e[j] = 0.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < 16; ++j) e[j] *= d[j] - delta;
+            bf16x8 f[2];
+            at_pack(f, e);
+#pragma unroll
+            for (int st = 0; st < 2; ++st)
+#pragma unroll
+                for (int db = 0; db < 2; ++db) dq[db] = at_mma(at_col_frag(K, db * 32, kb * 2 + st, lane), f[st], dq[db]);
         }
         if (more) {
-            at_store_tile(ks_[(t + 1) & 1], kr);
-            at_store_tile(vs_[(t + 1) & 1], vr);
+            at_store_tile(ks_ + ((t + 1) & 1) * TILE, kr);
+            at_store_tile(vs_ + ((t + 1) & 1) * TILE, vr);
         }
         __syncthreads();
+    }
+    if constexpr (HALVES) {   // the two waves of a row: the first one adds up and goes on
+        float *const acc = reinterpret_cast<float *>(tiles) + (wave & 1) * 2048;
+        if (half) {
+            at_put(acc, dq[0], lane);
+            at_put(acc + 1024, dq[1], lane);
+        }
+        __syncthreads();
+        if (half) return;
+        at_add(dq[0], acc, lane);
+        at_add(dq[1], acc + 1024, lane);
     }
     const int64_t at = ((int64_t)b * T + (row < T ? row : T - 1)) * ld3 + h * HD;
     at_row_grad(row < T ? p.dqkv + at : nullptr, p.qkv + at, p.table + (int64_t)(row < T ? row : T - 1) * 64, dq, p.eps, g);
 }
 
-__global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(AttnParams p)
+template <bool HALVES> __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(AttnParams p)
 {
-    __shared__ __align__(16) bf16_t qs_[2][AT_TILE * HD], ds_[2][AT_TILE * HD];
+    __shared__ __align__(16) bf16_t tiles[4][AT_TILE * HD];   // Q, Q, dY, dY
+    bf16_t *const qs_ = tiles[0], *const ds_ = tiles[2];
+    constexpr int TILE = AT_TILE * HD;
     __shared__ __align__(16) float ls_[2][AT_TILE], dl_[2][AT_TILE];
     int bh, b, h, rank;
     at_block(p, bh, b, h, rank);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, g = lane >> 5;
-    const int m0 = rank * AT_ROWS, n0 = m0 + wave * 32, T = p.T;   // n0: the wave's first kv row
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = HALVES ? wave >> 1 : 0, r = lane & 31, g = lane >> 5;
+    constexpr int ROWS = HALVES ? 64 : 128;
+    const int m0 = rank * ROWS, n0 = m0 + (HALVES ? wave & 1 : wave) * 32, T = p.T;   // n0: the wave's first kv row
     const int64_t ld3 = (int64_t)3 * p.H * HD, ld1 = (int64_t)p.H * HD;
     const TileSource qg(p.q + (int64_t)bh * T * HD, HD, T), kg(p.k + (int64_t)bh * T * HD, HD, T);
     const TileSource vg(p.qkv + (int64_t)b * T * ld3 + (2 * p.H + h) * HD, ld3, T), dg(p.dy + (int64_t)b * T * ld1 + h * HD, ld1, T);
@@ -446,13 +495,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(AttnParams p)
     qg.tile(qr, t0 * AT_TILE);
     dg.tile(dr, t0 * AT_TILE);
     load_row(t0);
-    at_store_tile(qs_[t0 & 1], qr);
-    at_store_tile(ds_[t0 & 1], dr);
+    at_store_tile(qs_ + (t0 & 1) * TILE, qr);
+    at_store_tile(ds_ + (t0 & 1) * TILE, dr);
     store_row(t0 & 1);
     __syncthreads();
     f32x16 dk[2] = {zero16(), zero16()}, dv[2] = {zero16(), zero16()};
     for (int t = t0; t < nt; ++t) {
-        const bf16_t *Q = qs_[t & 1], *D = ds_[t & 1];
+        const bf16_t *Q = qs_ + (t & 1) * TILE, *D = ds_ + (t & 1) * TILE;
         const float *L = ls_[t & 1], *E = dl_[t & 1];
         const bool more = t + 1 < nt;
         const int q0 = t * AT_TILE;
@@ -461,57 +510,71 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(AttnParams p)
             dg.tile(dr, q0 + AT_TILE);
             load_row(t + 1);
         }
-        if (q0 + AT_TILE - 1 >= n0) {
 #pragma unroll
-            for (int qb = 0; qb < 2; ++qb) {
-                f32x16 s = zero16(), d = zero16();
+        for (int i = 0; i < (HALVES ? 1 : 2); ++i) {
+            const int qb = HALVES ? half : i;
+            if (q0 + qb * 32 + 31 < n0) continue;   // past the diagonal
+            f32x16 s = zero16(), d = zero16();
 #pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-                    s = at_mma(at_row_frag(Q, qb * 32, ks, lane), kf[ks], s);
-                    d = at_mma(at_row_frag(D, qb * 32, ks, lane), vf[ks], d);
-                }
-                float e[16], u[16];
-#pragma unroll
-                for (int jq = 0; jq < 4; ++jq) {
-                    const f32x4 l4 = *reinterpret_cast<const f32x4 *>(L + qb * 32 + 8 * jq + 4 * g);
-                    const f32x4 e4 = *reinterpret_cast<const f32x4 *>(E + qb * 32 + 8 * jq + 4 * g);
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        const int j = jq * 4 + c;
-                        e[j] = __builtin_amdgcn_exp2f(fmaf(s[j], AT_EXP2, -l4[c]));
-                        u[j] = d[j] - e4[c];
-                    }
-                }
-                if (q0 + qb * 32 < n0 + 31) {   // reaches past the diagonal
-#pragma unroll
-                    for (int j = 0; j < 16; ++j)
-                        if (q0 + qb * 32 + at_row(j, g) < n0 + r) e[j] = 0.0f;
-                }
-#pragma unroll
-                for (int j = 0; j < 16; ++j) u[j] *= e[j];
-                bf16x8 f[2], w[2];
-                at_pack(f, e);
-                at_pack(w, u);
-#pragma unroll
-                for (int st = 0; st < 2; ++st)
-#pragma unroll
-                    for (int db = 0; db < 2; ++db) {
-                        dv[db] = at_mma(at_col_frag(D, db * 32, qb * 2 + st, lane), f[st], dv[db]);
-                        dk[db] = at_mma(at_col_frag(Q, db * 32, qb * 2 + st, lane), w[st], dk[db]);
-                    }
+            for (int ks = 0; ks < 4; ++ks) {
+                s = at_mma(at_row_frag(Q, qb * 32, ks, lane), kf[ks], s);
+                d = at_mma(at_row_frag(D, qb * 32, ks, lane), vf[ks], d);
             }
+            float e[16], u[16];
+#pragma unroll
+            for (int jq = 0; jq < 4; ++jq) {
+                const f32x4 l4 = *reinterpret_cast<const f32x4 *>(L + qb * 32 + 8 * jq + 4 * g);
+                const f32x4 e4 = *reinterpret_cast<const f32x4 *>(E + qb * 32 + 8 * jq + 4 * g);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const int j = jq * 4 + c;
+                    e[j] = __builtin_amdgcn_exp2f(fmaf(s[j], AT_EXP2, -l4[c]));
+                    u[j] = d[j] - e4[c];
+                }
+            }
+            if (q0 + qb * 32 < n0 + 31) {   // reaches past the diagonal
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    if (q0 + qb * 32 + at_row(j, g) < n0 + r) e[j] = 0.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < 16; ++j) u[j] *= e[j];
+            bf16x8 f[2], w[2];
+            at_pack(f, e);
+            at_pack(w, u);
+#pragma unroll
+            for (int st = 0; st < 2; ++st)
+#pragma unroll
+                for (int db = 0; db < 2; ++db) {
+                    dv[db] = at_mma(at_col_frag(D, db * 32, qb * 2 + st, lane), f[st], dv[db]);
+                    dk[db] = at_mma(at_col_frag(Q, db * 32, qb * 2 + st, lane), w[st], dk[db]);
+                }
         }
         if (more) {
-            at_store_tile(qs_[(t + 1) & 1], qr);
-            at_store_tile(ds_[(t + 1) & 1], dr);
+            at_store_tile(qs_ + ((t + 1) & 1) * TILE, qr);
+            at_store_tile(ds_ + ((t + 1) & 1) * TILE, dr);
             store_row((t + 1) & 1);
         }
         __syncthreads();
     }
+    if constexpr (HALVES) {   // the two waves of a row: one finishes dk, the other one dv
+        float *const acc = reinterpret_cast<float *>(tiles);
+#pragma unroll
+        for (int db = 0; db < 2; ++db) at_put(acc + wave * 2048 + db * 1024, half ? dk[db] : dv[db], lane);
+        __syncthreads();
+        const float *const other = acc + (wave ^ 2) * 2048;
+        if (half) {
+            at_add(dv[0], other, lane);
+            at_add(dv[1], other + 1024, lane);
+        } else {
+            at_add(dk[0], other, lane);
+            at_add(dk[1], other + 1024, lane);
+        }
+    }
     const int row = n0 + r;
     const int64_t at = ((int64_t)b * T + (row < T ? row : T - 1)) * ld3 + (p.H + h) * HD;
-    at_row_grad(row < T ? p.dqkv + at : nullptr, p.qkv + at, p.table + (int64_t)(row < T ? row : T - 1) * 64, dk, p.eps, g);
-    if (row >= T) return;
+    if (!HALVES || half == 0) at_row_grad(row < T ? p.dqkv + at : nullptr, p.qkv + at, p.table + (int64_t)(row < T ? row : T - 1) * 64, dk, p.eps, g);
+    if (row >= T || (HALVES && half == 0)) return;
     bf16_t *out = p.dqkv + at + (int64_t)p.H * HD;
 #pragma unroll
     for (int db = 0; db < 2; ++db)
@@ -525,10 +588,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(AttnParams p)
 static int check_attn(const char *who, int64_t B, int64_t T, int64_t H)
 {
     if (B <= 0 || T <= 0 || H <= 0) return set_error(RDB_E_SHAPE, "%s: sizes must be positive", who);
-    if (T > (1 << 20) || H > 1024 || T * 3 * H * HD * 2 >= (1ll << 30) || B * H * cdiv(T, AT_ROWS) >= (1ll << 31))
+    if (T > (1 << 20) || H > 1024 || T * 3 * H * HD * 2 >= (1ll << 30) || B * H * cdiv(T, 128) >= (1ll << 31))
         return set_error(RDB_E_UNSUPPORTED, "%s: a sequence's qkv must stay below 2^30 bytes", who);
     return RDB_OK;
 }
+// us with blocks of 128 rows -> of 64, batch x heads x tokens: forward with preparation 1 x 12 x 1024 25.2 -> 21.3, 8 x 10 x 1024 (640
+// blocks of 128) 34.0 -> 32.8, 8 x 12 x 1024 (768) 36.7 -> 39.0; backward 1 x 12 x 1024 49.6 -> 33.1, 4 x 12 x 1024 (384) 54.3 -> 47.3, 7 x 8 x 1024
+// (448) 54.7 -> 57.3.
+static bool at_halves(const AttnParams &p, bool backward) { return cdiv(p.T, 128) * p.BH <= (backward ? 384 : 640); }
 static bool at16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace rdb
@@ -559,8 +626,10 @@ extern "C" int rdb_causal_attention_fwd(void *y, void *q, void *k, float *scratc
     p.T = (int)T;
     p.H = (int)heads;
     p.BH = (int)(batch * heads);
-    p.nb = (int)cdiv(T, AT_ROWS);
-    attn_fwd_kernel<<<(unsigned)(p.nb * p.BH), 256, 0, s>>>(p);
+    const bool halves = at_halves(p, false);
+    p.nb = (int)cdiv(T, halves ? 64 : 128);
+    if (halves) attn_fwd_kernel<true><<<(unsigned)(p.nb * p.BH), 256, 0, s>>>(p);
+    else attn_fwd_kernel<false><<<(unsigned)(p.nb * p.BH), 256, 0, s>>>(p);
     return check_launch("attn_fwd_kernel");
 }
 
@@ -585,11 +654,14 @@ extern "C" int rdb_causal_attention_bwd(void *dqkv, const void *dy, const void *
     p.T = (int)T;
     p.H = (int)heads;
     p.BH = (int)(batch * heads);
-    p.nb = (int)cdiv(T, AT_ROWS);
+    const bool halves = at_halves(p, true);
+    p.nb = (int)cdiv(T, halves ? 64 : 128);
     p.eps = eps;
     const unsigned grid = (unsigned)(p.nb * p.BH);
-    attn_bwd_dq_kernel<<<grid, 256, 0, s>>>(p);
+    if (halves) attn_bwd_dq_kernel<true><<<grid, 256, 0, s>>>(p);
+    else attn_bwd_dq_kernel<false><<<grid, 256, 0, s>>>(p);
     if (int rc = check_launch("attn_bwd_dq_kernel")) return rc;
-    attn_bwd_dkv_kernel<<<grid, 256, 0, s>>>(p);
+    if (halves) attn_bwd_dkv_kernel<true><<<grid, 256, 0, s>>>(p);
+    else attn_bwd_dkv_kernel<false><<<grid, 256, 0, s>>>(p);
     return check_launch("attn_bwd_dkv_kernel");
 }

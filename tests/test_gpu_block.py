@@ -179,6 +179,12 @@ def test_causal_attention(ext, B, T, H, inv):
     assert torch.equal(y2, ya) and torch.equal(torch.autograd.grad(y2, a, dy)[0], ga)
 
 
+# enough blocks for 128 rows each: forward and backward, backward alone, with two blocks to a head
+@pytest.mark.parametrize("B,T,H,inv", [(8, 1100, 9, "bf16"), (5, 900, 11, "fp32"), (43, 129, 8, "bf16")])
+def test_causal_attention_of_many_rows(ext, B, T, H, inv):
+    test_causal_attention(ext, B, T, H, inv)
+
+
 def test_model_with_and_without_the_fused_kernels(ext, monkeypatch):
     from randumb_amd import gpt
 

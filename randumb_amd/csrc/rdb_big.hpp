@@ -280,25 +280,23 @@ __device__ __forceinline__ void big_store_bf16(f32x16 (&acc)[BM / 64][BN / 64], 
     static_assert(PIECES % GROUP == 0, "pieces leave in groups of 8");
     const int a = (t % (BM / 8)) * 8, bq = t / (BM / 8);   // 256 % (BM / 8) == 0: a thread's pieces share their columns
     const bool a_ok = a0 + a < na;
+    // Streaming stores also where rows are not whole lines of 128 bytes (16 bytes a lane, most lines whole): without, a forward pass alone is
+    // faster (6000 tokens x 512 -> 6008, k = 320: 61.7 -> 59.5 us) but y, 72 MB, takes the place of what the backward pass reads (step 169 -> 181).
     // eight pieces are read from LDS before the first of them is stored: one wait for LDS per group instead of one per piece
-    auto pieces = [&](auto stream) __attribute__((always_inline)) {
 #pragma unroll
-        for (int p0 = 0; p0 < PIECES; p0 += GROUP) {
-            f32x4 v[GROUP];
+    for (int p0 = 0; p0 < PIECES; p0 += GROUP) {
+        f32x4 v[GROUP];
 #pragma unroll
-            for (int q = 0; q < GROUP; ++q) v[q] = *reinterpret_cast<const f32x4 *>(lds + ((p0 + q) * (256 / (BM / 8)) + bq) * LDS_LD + a);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int q = 0; q < GROUP; ++q) v[q] = *reinterpret_cast<const f32x4 *>(lds + ((p0 + q) * (256 / (BM / 8)) + bq) * LDS_LD + a);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int q = 0; q < GROUP; ++q) {
-                const int b = (p0 + q) * (256 / (BM / 8)) + bq;
-                const uint32_t off = (a_ok && b0 + b < nb) ? (uint32_t)(((int64_t)(b0 + b) * ld + a0 + a) * 2) : BUFFER_OOB;
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v[q]), rs, (int)off, 0, decltype(stream)::value ? 2 : 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
+        for (int q = 0; q < GROUP; ++q) {
+            const int b = (p0 + q) * (256 / (BM / 8)) + bq;
+            const uint32_t off = (a_ok && b0 + b < nb) ? (uint32_t)(((int64_t)(b0 + b) * ld + a0 + a) * 2) : BUFFER_OOB;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v[q]), rs, (int)off, 0, STREAM ? 2 : 0);
         }
-    };
-    if (STREAM && ld % 64 == 0) pieces(std::true_type{});   // rows of whole lines only: see f32_gemm_block
-    else pieces(std::false_type{});
+        __builtin_amdgcn_sched_barrier(0);
+    }
     __syncthreads();
 }
 

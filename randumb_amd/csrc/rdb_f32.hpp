@@ -379,7 +379,7 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false, int ES = 4> struct Fg
 // Results leave with streaming stores: they would be written back from L2 at the end of the kernel otherwise, after the last
 // block (y of that layer, 25 MB: 26.4 -> 24.8 us).  Not so where rows are not whole lines of 128 bytes: a streaming store of part of
 // a line goes to memory as such, where L2 puts a line's parts together (y of 3899 tokens x 5603, k = 199: 107 -> 75 us; 1500 x 5245, k =
-// 156: 36 -> 24.6; 4096 x 999, k = 100: 16.7 -> 15.3; on the tiles of rdb_big.hpp in bf16 6000 x 512 -> 6008, k = 320: 61.7 -> 59.5).
+// 156: 36 -> 24.6; 4096 x 999, k = 100: 16.7 -> 15.3; the step of 4096 x 1024 -> 8190, k = 128: 275 -> 267).
 // AES, BES: bytes per element of the two matrices (SPLIT: 4, or 2, bf16; otherwise 0, see FgOperand).
 // f32_gemm_block: what block (bx, by, bz) of a product does (gx: how many there are along x).  `lds`: FgBlock::LDS floats; not_finite: a
 // word of LDS.

@@ -21,9 +21,10 @@
 //
 // Measured at 8 sequences x 12 heads x 1024 tokens, us: forward 36.7 (13.5 of them prep), backward 79 (the stock operators they
 // replace: attention 81 forward, 267 backward, normalisation and rotation some 450).  13 GFLOP forward and 45 backward.  No pipe is
-// full (SQ counters, shares of a compute unit's time): matrix cores 24 to 29 %, vector ALU 42 to 48 % (25 % of the
-// forward pass in exponentials, 16 a lane for 16 matrix instructions), LDS 32 to 41 % without bank conflicts; two waves a SIMD and a
-// barrier per 64 rows put them one after the other.  The preparing kernel is the vector ALU's (81 %).
+// full (SQ counters, shares of a compute unit's time): matrix cores 28 to 30 %, vector ALU 40 to 51 % (29 % of the
+// forward pass in exponentials, 16 a lane for 16 matrix instructions), LDS 36 to 43 % without bank conflicts; two waves a SIMD and a
+// barrier per 64 rows put them one after the other.  The preparing kernel is the vector ALU's (94 %;
+// without its 64-bit divisions by T and with one call for sine and cosine it is 1 us shorter, which no step showed).
 #include "rdb_gemm.hpp"
 
 namespace rdb {

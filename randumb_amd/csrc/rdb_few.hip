@@ -461,47 +461,17 @@ template <typename E, int KS, int TC, int TE> __global__ __launch_bounds__(256, 
 }
 
 // ----------------------------------------------------------------------------------------------- host side
-// Where these kernels are ahead of those of rdb_smallk.hip, rdb_factored.hip and rdb_f32.hip.  `units` are the expanding blocks of one
-// tile of tokens: each splits its tokens' z again, so the more of them there are, and the larger k, the sooner the kernels that
-// make z once for wide tiles win; fp32 multiplies twice as much.  us per call, those kernels -> here:
-//   k <= 64    128 x 2048 -> 2048, k = 64: bf16 16.1 -> 9.1, fp32 17.1 -> 10.0; 128 x 3000 -> 11008, k = 64 (1376 units): 18.9 ->
-//              14.1 and 19.6 -> 16.8; 256 x 8192 -> 8192 (2048): fp32 24.4 -> 27.9
-//   k <= 128   128 x 8192 -> 8192: bf16 25.8 -> 18.3, fp32 25.1 -> 22.3 (1024 units); 192 (1536): 29.7 -> 23.1, fp32 26.1 -> 30.0
-//   k <= 256   128 x 4096 -> 4096: bf16 20.9 -> 18.5, fp32 24.6 -> 22.2 (512 units); 160 (640): 22.4 -> 23.0 and 25.6 -> 30.5;
-//              96 x 4096 -> 11008: 39 -> 22.3 and 39.4 -> 32.1; fp32 48 x 5000 -> 600, k = 200: 16.6 -> 19.1
-//   beyond     64 x 1024 -> 4096, k = 512: bf16 17.8 -> 16.0; 64 x 1504 -> 6000, k = 304 (376 units): 17.1 -> 18.5;
-//              fp32 32 x 8192 -> 11008, k = 512: 39 -> 33, 48 tokens 33 -> 50
-// bf16 contractions of at most 512 are short for the kernels of rdb_factored.hip too: 160 x 384 -> 8000, k = 24 (1250 units): 10.7 -> 11.1;
-// 128 x 512 -> 4096, k = 256 (512 units): 12.8 -> 13.1; 64 tokens (256): 12.4 -> 10.1.
-// 256 tokens are the most all the same, though 512 x 768 -> 3072, k = 64 would be 13.4 -> 12.7 (fp32 16.8 -> 15.0): beyond, y stays bit
-// for bit that of the forms that keep z for a backward pass.
-// The factored form is taken as far as everywhere: up to 16 times the products of one with a stored weight.
-static bool few_pays(const rdb_linear_desc *d)
-{
-    const int64_t T = d->tokens, k = d->k, units = cdiv(d->out_f, FEW_ROWS) * cdiv(T, 16);
-    const bool b16 = d->act_dtype == RDB_BF16;
-    if (T <= 16) return true;
-    if (T > FEW_TOKENS) return false;
-    if (b16 && d->in_f <= 512 && units > (k <= 128 ? 512 : 256)) return false;
-    if (k <= 128) return units <= (b16 || k <= 64 ? 1536 : 1024);
-    if (k > 256) return T <= 32 || (b16 && T <= 96 && units <= 300);
-    return b16 ? T <= 96 || units <= 512 : (T <= 96 || (T <= 192 && units <= 512)) && d->in_f <= 4 * d->out_f;
-}
-static bool few_ok(const rdb_linear_desc *d)
-{
-    const bool f32 = d->act_dtype == RDB_F32 && d->coef_dtype == RDB_F32, b16 = d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16;
-    return (f32 || b16) && d->algo == RDB_ALGO_AUTO && d->coef_rows != 0 && d->k > 0 && d->k <= FEW_K && d->tokens > 0 && d->in_f > 0 &&
-           d->out_f > 0 && d->in_f < (1 << 20) && d->out_f < (1 << 24) && few_pays(d) && d->k * (d->in_f + d->out_f) < 16 * d->in_f * d->out_f;
-}
 // Chunks: about eight of them (sixteen where there is one range of coefficients), of 128 to 512 values (a contracting block hashes a chunk for 16 coefficients: 128 values cost it 0.6 us;
 // an expanding block reads eight at a time: 1 x 4096 -> 4096, k = 16: chunks of 128, 256, 512, 1024: 8.9, 8.0, 8.2, 10.9 us).
 // te: tiles of an expanding block.  Finer is sooner ready while the blocks run side by side, two (of k > 128: one) to a compute unit: 64 x
 // 768 -> 3072, k = 64: 8.2 us, two tiles 9.1; 80 x 8192 -> 8192, k = 64, 640 blocks of one tile: 18.7, two tiles 15.1.
 // sum: beyond 200 KB of partial sums for a block they are added up once, by a launch of its own, and not by every expanding block
 // (48 to a block, 32 tokens x 4096 -> 11008, k = 256: 15.6 -> 14.9 us; 16 tokens, 131 KB: 11.5, and 12.7 with it).
-// one: a single launch where the expanding blocks are few and the partial sums small; tags and reads that go around L2 cost many
-// blocks more than a launch does (5 x 1001 -> 999, k = 99: two launches 9.2, one 7.5; 16 x 4096 -> 11008, k = 256: 11.5 and 13.5; 1 x 4096
-// -> 4096, k = 16: 8.0 and 8.6, but a program's host takes 10.7 to issue two).
+// one: a single launch where the expanding blocks are few and the partial sums of each small; tags and reads that go around L2 cost many
+// blocks more than a launch does (16 x 4096 -> 11008, k = 256: two launches 11.5, one 13.5), but a program's host takes 10.7 us to issue two.
+// us of a program's call, two launches -> one: 5 x 1001 -> 999, k = 99: 9.2 -> 7.5 (library calls); 100 x 264 -> 352, k = 64, 42 blocks: 11.0 ->
+// 8.6; 32 x 1024 -> 2048, k = 128, 64 blocks of 64 KB: 10.8 -> 9.2; 4 x 2048 -> 10000, k = 32, 157 blocks: 10.8 -> 9.1; 64 x 768 -> 2048, k = 64, 128
+// blocks: 10.9 -> 10.0; 256 x 512 -> 640, k = 128, fp32, 160 blocks of 32 KB: 11.2 -> 11.7.
 struct FewPlan {
     int wave_values, chunks, ranges;
     int tile, tiles, tc, te;
@@ -530,10 +500,47 @@ static FewPlan few_plan(const rdb_linear_desc *d)
     f.part_bytes = f.chunks * per_chunk * f.tiles;
     f.c_blocks = (int)(f.chunks * f.ranges * c_groups);
     f.e_blocks = (int)(rows * cdiv(f.tiles, f.te));
-    f.one = !f.sum && ((f.e_blocks <= 32 && f.part_bytes <= 100 * 1024) || (f.e_blocks <= 80 && f.part_bytes <= 32 * 1024));
+    const int64_t block_bytes = f.chunks * per_chunk * std::min(f.te, f.tiles);   // what an expanding block reads
+    f.one = !f.sum && ((f.e_blocks <= 64 && block_bytes <= 100 * 1024) || (f.e_blocks <= 160 && block_bytes <= 32 * 1024));
     return f;
 }
 
+// Where these kernels are ahead of those of rdb_smallk.hip, rdb_factored.hip and rdb_f32.hip.  `units` are the expanding blocks of one
+// tile of tokens: each splits its tokens' z again, so the more of them there are, and the larger k, the sooner the kernels that
+// make z once for wide tiles win; fp32 multiplies twice as much.  us per call, those kernels -> here:
+//   k <= 64    128 x 2048 -> 2048, k = 64: bf16 16.1 -> 9.1, fp32 17.1 -> 10.0; 128 x 3000 -> 11008, k = 64 (1376 units): 18.9 ->
+//              14.1 and 19.6 -> 16.8; 256 x 8192 -> 8192 (2048): fp32 24.4 -> 27.9
+//   k <= 128   128 x 8192 -> 8192: bf16 25.8 -> 18.3, fp32 25.1 -> 22.3 (1024 units); 192 (1536): 29.7 -> 23.1, fp32 26.1 -> 30.0
+//   k <= 256   128 x 4096 -> 4096: bf16 20.9 -> 18.5, fp32 24.6 -> 22.2 (512 units); 160 (640): 22.4 -> 23.0 and 25.6 -> 30.5;
+//              96 x 4096 -> 11008: 39 -> 22.3 and 39.4 -> 32.1; fp32 48 x 5000 -> 600, k = 200: 16.6 -> 19.1
+//   beyond     64 x 1024 -> 4096, k = 512: bf16 17.8 -> 16.0; 64 x 1504 -> 6000, k = 304 (376 units): 17.1 -> 18.5;
+//              fp32 32 x 8192 -> 11008, k = 512: 39 -> 33, 48 tokens 33 -> 50
+// bf16 contractions of at most 512 are short for the kernels of rdb_factored.hip too, which take one launch where a program's host needs 10.7 us
+// for two (no gradients wanted; 128 x 320 -> 640, k = 160: 10.2 -> 11.0): 160 x 384 -> 8000, k = 24 (1250 units): 10.7 -> 11.1;
+// 128 x 512 -> 4096, k = 256 (512 units): 12.8 -> 13.1; 64 tokens (256): 12.4 -> 10.1.
+// Beyond 256 tokens only contractions of 512 and more, where the other kernels' one block a tile takes longest: 512 x 2048 -> 2048, k = 64: 19.0 ->
+// 13.2, fp32 18.5 -> 15.1; 512 x 8192 -> 512, k = 16: 30.9 -> 11.5 and 21.1 -> 13.0; 512 x 4096 -> 512, k = 128: 28.7 -> 18.9, fp32 24.0 -> 24.6; 512 x
+// 520 -> 2000, k = 64: 12.0 -> 11.2; 640 tokens x 1001 -> 999, k = 60: 16.2 -> 17.4.  For shorter ones y stays bit for bit that of the forms that keep z.
+// The factored form is taken as far as everywhere: up to 16 times the products of one with a stored weight.
+static bool few_pays(const rdb_linear_desc *d)
+{
+    const int64_t T = d->tokens, k = d->k, units = cdiv(d->out_f, FEW_ROWS) * cdiv(T, 16);
+    const bool b16 = d->act_dtype == RDB_BF16;
+    if (T > 2 * FEW_TOKENS) return false;
+    if (b16 && d->in_f < 512 && (T > 96 || k > 64) && !few_plan(d).one) return false;
+    if (T <= 16) return true;
+    if (T > (d->in_f >= 512 && (k <= 64 || (b16 && k <= 128)) ? 2 * FEW_TOKENS : FEW_TOKENS)) return false;
+    if (b16 && d->in_f <= 512 && units > (k <= 128 ? 512 : 256)) return false;
+    if (k <= 128) return units <= (b16 || k <= 64 ? 1536 : 1024);
+    if (k > 256) return T <= 32 || (b16 && T <= 96 && units <= 300);
+    return b16 ? T <= 96 || units <= 512 : (T <= 96 || (T <= 192 && units <= 512)) && d->in_f <= 4 * d->out_f;
+}
+static bool few_ok(const rdb_linear_desc *d)
+{
+    const bool f32 = d->act_dtype == RDB_F32 && d->coef_dtype == RDB_F32, b16 = d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16;
+    return (f32 || b16) && d->algo == RDB_ALGO_AUTO && d->coef_rows != 0 && d->k > 0 && d->k <= FEW_K && d->tokens > 0 && d->in_f > 0 &&
+           d->out_f > 0 && d->in_f < (1 << 20) && d->out_f < (1 << 24) && few_pays(d) && d->k * (d->in_f + d->out_f) < 16 * d->in_f * d->out_f;
+}
 int64_t linear_few_workspace(const rdb_linear_desc *d)
 {
     if (!few_ok(d)) return 0;

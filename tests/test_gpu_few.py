@@ -29,7 +29,8 @@ def _rel(a, b):
                                             (33, 300, 100, 33), (48, 264, 2112, 64), (48, 4100, 300, 250), (47, 1200, 520, 510),
                                             # one tile of tokens and two to an expanding block, the last group not full
                                             (49, 130, 65, 17), (97, 264, 5100, 40), (96, 260, 2800, 256), (81, 515, 130, 129), (90, 700, 2850, 300),
-                                            (192, 2050, 1000, 131), (256, 1001, 999, 100), (240, 600, 3000, 16), (255, 264, 352, 64)])
+                                            (192, 2050, 1000, 131), (256, 1001, 999, 100), (240, 600, 3000, 16), (255, 264, 352, 64), (512, 512, 600, 64),
+                                            (500, 1030, 200, 30), (509, 2000, 2200, 50)])
 def test_against_float64(T, in_f, out_f, k, dtype):
     print(f"case few T={T} in={in_f} out={out_f} k={k} {dtype}", flush=True)
     x, c, b, N = _case(T, in_f, out_f, k, dtype)
@@ -77,7 +78,7 @@ def test_not_finite(k, dtype):
 
 def test_recorded_launches():
     """Both forms recorded into one graph and replayed on changing inputs, with eager calls in between."""
-    shapes = [(5, 1001, 999, 99), (16, 4096, 4096, 256), (40, 4096, 512, 256)]   # one launch, two, three
+    shapes = [(5, 1001, 999, 99), (100, 264, 352, 64), (16, 4096, 4096, 256), (40, 8192, 512, 512)]   # one launch (one group of tokens, four), two, three
     cases = [_case(*s, torch.bfloat16)[:2] for s in shapes]
     call = lambda: [hip.linear_fwd(x, c, s[1], s[2], s[1], 1, 5) for s, (x, c) in zip(shapes, cases)]
     call()
@@ -94,8 +95,8 @@ def test_recorded_launches():
         torch.cuda.synchronize()
 
 
-# 20 and 64 tokens: these kernels, one group of tokens and several; 264: the vector-ALU kernels of rdb_smallk.hip, whose wait is their own
-@pytest.mark.parametrize("T", [20, 64, 264])
+# 20 and 64 tokens: these kernels, one group of tokens and several; 520: the vector-ALU kernels of rdb_smallk.hip, whose wait is their own
+@pytest.mark.parametrize("T", [20, 64, 520])
 def test_a_wait_that_gives_up(T):
     """NaN throughout, the counter, and the host's watch, as for the other one-launch forms."""
     in_f, out_f, k = 1000, 520, 16

@@ -55,7 +55,8 @@ constexpr int COEF_CHUNK = 2048;
 // term by term.  Without it, and with MAT_UNROLL terms a turn of the loop (still one after the other), a term takes 17 vector instructions
 // instead of 19: 768 x 3072 elements, k = 256: 219 -> 205 us, and the pass of that layer, 1024 tokens, 538 -> 520; 4096 rows of a 50304 x
 // 768 table, forward and backward, 525 -> 522 (one term a turn: 540).  The round constants stay literals: in scalar or vector registers the
-// same instructions take 2 to 6 % longer.
+// same instructions take 2 to 6 % longer.  What is left of a chunk goes by fours and twos: 618 x 2480 elements, k = 23, 21.2 -> 20.9 us (with the
+// factor term by term and without the look at the coefficients 19.9: at so few terms the look is not paid back).
 constexpr float MAT_LARGE = 3.777893186295716e22f;   // 2^75
 constexpr int MAT_UNROLL = 8;
 
@@ -106,17 +107,22 @@ template <bool GATHER, int LANES> __global__ __launch_bounds__(NT) void material
             float sum = acc * 2147483648.0f;
             int j = part;
             if (LANES == 1) {
-                for (; j + MAT_UNROLL <= cnt; j += MAT_UNROLL) {
-                    float c[MAT_UNROLL];
+                auto turn = [&](auto terms) __attribute__((always_inline)) {
+                    constexpr int TERMS = decltype(terms)::value;
+                    float c[TERMS];
 #pragma unroll
-                    for (int e = 0; e < MAT_UNROLL; ++e) c[e] = cs[j + e];
+                    for (int e = 0; e < TERMS; ++e) c[e] = cs[j + e];
 #pragma unroll
-                    for (int e = 0; e < MAT_UNROLL; ++e) {
+                    for (int e = 0; e < TERMS; ++e) {
                         sum = fmaf((float)(int32_t)sq5_tail_apart(first), c[e], sum);
                         first += SQ5_N1;
                         __builtin_amdgcn_sched_barrier(0);   // one term after the other
                     }
-                }
+                    j += TERMS;
+                };
+                while (j + MAT_UNROLL <= cnt) turn(std::integral_constant<int, MAT_UNROLL>{});
+                if (j + 4 <= cnt) turn(std::integral_constant<int, 4>{});
+                if (j + 2 <= cnt) turn(std::integral_constant<int, 2>{});
             }
             for (; j < cnt; j += LANES) {
                 sum = fmaf((float)(int32_t)sq5_tail_apart(first), cs[j], sum);

@@ -15,6 +15,7 @@
 #include <torch/csrc/autograd/autograd.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -311,6 +312,43 @@ std::pair<Tensor, Tensor> linear_bwd_dcoef(const Tensor &dy0, const Tensor &x0, 
 
 rdb_linear_desc rbias_desc(const Tensor &rows, const Layer &l) { return desc(rows.size(0), l, 8, l.out_f, at::kBFloat16, at::kBFloat16); }
 
+// First derivatives that a function's backward pass computes under create_graph without a graph, having no second ones: they are there,
+// and going through them again raises (a result without a graph would pass for one that depends on nothing).  dy: the incoming
+// gradient; inputs: which of the function's tensor inputs the derivative depends on.  The raising node leads to what these come
+// from, so that it is on the way to all of them, whichever of them a derivative is asked for.
+Tensor once_differentiable(const char *who, const Tensor &grad, const Tensor &dy, std::initializer_list<int> inputs)
+{
+    if (!at::GradMode::is_enabled() || !grad.defined()) return grad;
+    torch::autograd::edge_list edges;
+    auto depends_on = [&](const torch::autograd::Edge &e) {
+        if (e.is_valid()) edges.push_back(e);
+    };
+    if (dy.requires_grad()) depends_on(torch::autograd::impl::gradient_edge(dy));
+    const auto node = torch::autograd::get_current_node();
+    for (int i : inputs)
+        if (node && i >= 0 && i < (int)node->num_outputs()) depends_on(node->next_edge(i));
+    if (edges.empty()) return grad;   // a constant
+    const Tensor out = grad.detach();
+    torch::autograd::set_history(out, std::make_shared<torch::autograd::Error>(std::string(who) + " has no second derivative", std::move(edges)));
+    return out;
+}
+// bias_grads under create_graph: linear in dy, by differentiable operators
+std::pair<Tensor, Tensor> bias_grads_with_graph(const Tensor &dy, const std::vector<int64_t> &m);
+// What a matrix-coef layer's backward pass returns, under create_graph too: dx depends on dy, the coefficients and the scale; dC and the scale's
+// gradient on dy and x.  x is input 0, the coefficients are 1, the scale is `scale` (negative: none).
+void layer_gradients(const Tensor &dy, int scale, Tensor &dx, Tensor &dc, Tensor &ds, std::pair<Tensor, Tensor> &db, const std::vector<int64_t> &bias)
+{
+    if (!at::GradMode::is_enabled()) return;
+    dx = once_differentiable("linear", dx, dy, {1, scale});
+    dc = once_differentiable("linear", dc, dy, {0});
+    ds = once_differentiable("linear", ds, dy, {0});
+    if (dy.requires_grad() && (db.first.defined() || db.second.defined())) {
+        const auto again = bias_grads_with_graph(dy, bias);
+        if (db.first.defined()) db.first = again.first;
+        if (db.second.defined()) db.second = again.second;
+    }
+}
+
 // ----------------------------------------------------------------------------------------------- one-call form
 // y = x.W^T (+ bias) with x saved; the three products of the layer as three calls, or, for the layers of which the library keeps
 // z = x.N^T (rdb_linear_kept_bytes), that saved and one call each way.
@@ -341,6 +379,14 @@ class OneCallLinear : public Function<OneCallLinear> {
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
+        Tensor dx, dc, ds;
+        std::pair<Tensor, Tensor> db;
+        gradients(ctx, grads, dx, dc, ds, db);
+        layer_gradients(grads[0], ctx->saved_data["layer"].toIntVector()[5] ? 2 : -1, dx, dc, ds, db, ctx->saved_data["bias"].toIntVector());
+        return {dx, dc, ds, db.first, db.second, Tensor(), Tensor()};
+    }
+    static void gradients(AutogradContext *ctx, const variable_list &grads, Tensor &dx, Tensor &dc, Tensor &dsb, std::pair<Tensor, Tensor> &db)
+    {
         const auto saved = ctx->get_saved_variables();
         const Tensor &x = saved[0], &coefs = saved[1], &sb = saved[2], &kept = saved[3];
         const auto m = ctx->saved_data["layer"].toIntVector();
@@ -354,7 +400,6 @@ class OneCallLinear : public Function<OneCallLinear> {
         const bool want_dx = ctx->needs_input_grad(0), want_dc = ctx->needs_input_grad(1);
         bool want_sb = has_sb && ctx->needs_input_grad(2);
         const Tensor dy = kept.defined() ? near_act(grads[0]) : grads[0].contiguous();
-        Tensor dx, dc, dsb;
         if (kept.defined()) {
             if (want_dx || want_dc || want_sb) {
                 const c10::OptionalDeviceGuard guard(dy.device());
@@ -372,8 +417,8 @@ class OneCallLinear : public Function<OneCallLinear> {
                       "rdb_linear_bwd_kept");
                 if (want_sb) dsb = dsb.to(sb.scalar_type());
             }
-            const auto db = bias_grads(ctx, dy, ctx->saved_data["bias"].toIntVector(), has_sb ? 3 : 2);
-            return {dx, dc, dsb, db.first, db.second, Tensor(), Tensor()};
+            db = bias_grads(ctx, dy, ctx->saved_data["bias"].toIntVector(), has_sb ? 3 : 2);
+            return;
         }
         if (want_dx && want_sb && l.sO == l.in_f && l.sI == 1) {
             // the random-bias product dy.R that dx needs anyway also gives the gradient of the bias's scale (reduced against x
@@ -391,8 +436,7 @@ class OneCallLinear : public Function<OneCallLinear> {
             dc = both.first.to(coefs.scalar_type());
             if (want_sb) dsb = both.second.to(sb.scalar_type());
         }
-        const auto db = bias_grads(ctx, dy, ctx->saved_data["bias"].toIntVector(), has_sb ? 3 : 2);
-        return {dx, dc, dsb, db.first, db.second, Tensor(), Tensor()};
+        db = bias_grads(ctx, dy, ctx->saved_data["bias"].toIntVector(), has_sb ? 3 : 2);
     }
 };
 
@@ -436,6 +480,15 @@ class ProjectedLinear : public Function<ProjectedLinear> {
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
+        Tensor dx, dc, ds;
+        std::pair<Tensor, Tensor> db;
+        gradients(ctx, grads, dx, dc, ds, db);
+        const auto m = ctx->saved_data["layer"].toIntVector();
+        layer_gradients(grads[0], m[3] ? (int)(2 + m[4]) : -1, dx, dc, ds, db, ctx->saved_data["bias"].toIntVector());
+        return {dx, dc, db.first, db.second, Tensor(), ds, Tensor()};
+    }
+    static void gradients(AutogradContext *ctx, const variable_list &grads, Tensor &dx, Tensor &dc, Tensor &dsb, std::pair<Tensor, Tensor> &db)
+    {
         const auto saved = ctx->get_saved_variables();
         const Tensor &state = saved[0], &coefs = saved[1], &scale_bias = saved[2];
         const auto m = ctx->saved_data["layer"].toIntVector();
@@ -459,7 +512,6 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         if (c.scalar_type() != dy.scalar_type()) fail(PyExc_RuntimeError, std::string(who) + ": the saved coefficients came back in another dtype");
         restored_values(who, state, dy, at::kByte, rdb_linear_projection_bytes(&d));
         void *s = stream_of(dy);
-        Tensor dx, dc, dsb;
         if (want_dc && (want_dx || f32)) {
             // bf16 coefficients: their gradient leaves the kernel that adds it up in bf16, where the layer runs as one chunk of tokens
             const bool to_bf16 = !f32 && rdb_linear_projection_chunks(&d, nullptr) == 1;
@@ -497,8 +549,7 @@ class ProjectedLinear : public Function<ProjectedLinear> {
             }
         }
         if (!want_x) dx = Tensor();
-        const auto db = bias_grads(ctx, dy, ctx->saved_data["bias"].toIntVector(), 2);
-        return {dx, dc, db.first, db.second, Tensor(), dsb, Tensor()};
+        db = bias_grads(ctx, dy, ctx->saved_data["bias"].toIntVector(), 2);
     }
 };
 
@@ -537,6 +588,14 @@ class CoefValues : public Function<CoefValues> {
         return {g[0].to((at::ScalarType)m[2]), m[3] >= 0 ? g[1].to((at::ScalarType)m[3]) : Tensor(), Tensor(), Tensor()};
     }
 };
+
+std::pair<Tensor, Tensor> bias_grads_with_graph(const Tensor &dy, const std::vector<int64_t> &m)
+{
+    const Tensor db = dy.sum(0, false, at::kFloat);
+    if (m[1] < 0) return {db.to((at::ScalarType)m[2]), Tensor()};
+    const auto g = CoefGrads::apply(db, m[0], m[1], m[3] >= 0);
+    return {g[0].to((at::ScalarType)m[2]), m[3] >= 0 ? g[1].to((at::ScalarType)m[3]) : Tensor()};
+}
 
 // out [M x N], contiguous, = A . B^T (+ bias); A [M x K], B [N x K], or stored transposed (across).  fp32: the library's own product;
 // bf16: torch's.  out is the caller's, because what an autograd function returns must not be a view (in-place changes of it are refused)
@@ -614,11 +673,8 @@ class VectorLinear : public Function<VectorLinear> {
                 if (want_s) ds = g[1].to((at::ScalarType)m[3]);
             }
             const auto bm = ctx->saved_data["bias"].toIntVector();
-            if (bm[0] < 0) return {dx, dc, ds, Tensor(), Tensor(), Tensor(), Tensor()};
-            const Tensor db = dy.sum(0);
-            if (bm[1] < 0) return {dx, dc, ds, db.to((at::ScalarType)bm[2]), Tensor(), Tensor(), Tensor()};
-            const auto g = CoefGrads::apply(db, bm[0], bm[1], bm[3] >= 0);
-            return {dx, dc, ds, g[0].to((at::ScalarType)bm[2]), bm[3] >= 0 ? g[1].to((at::ScalarType)bm[3]) : Tensor(), Tensor(), Tensor()};
+            const auto db = bm[0] < 0 ? std::pair<Tensor, Tensor>() : bias_grads_with_graph(dy, bm);
+            return {dx, dc, ds, db.first, db.second, Tensor(), Tensor()};
         }
         if (want_x) {
             const bool kept = saved[3].defined();
@@ -637,15 +693,6 @@ class VectorLinear : public Function<VectorLinear> {
     }
 };
 
-// First derivatives computed under create_graph by a function that has no second ones: the first ones are there, going through them
-// again raises (a result without a graph would pass for one that does not depend on the inputs).  varies: whether something the
-// derivative depends on has a gradient to come.
-Tensor once_differentiable(const char *who, const Tensor &grad, bool varies)
-{
-    if (!at::GradMode::is_enabled() || !varies) return grad;
-    auto error = std::make_shared<torch::autograd::DelayedError>(std::string(who) + " has no second derivative", 1);
-    return (*error)({grad.detach().set_requires_grad(true)})[0];
-}
 // Gradient of f(inputs...) with a graph of its own (create_graph), by f's stock operators.  Inputs without a gradient to come: undefined
 template <typename F> variable_list stock_gradient(F f, const variable_list &inputs, const variable_list &grads)
 {
@@ -689,7 +736,7 @@ class EmbedRows : public Function<EmbedRows> {
     {
         const Tensor idx = ctx->get_saved_variables()[0];
         const auto m = ctx->saved_data["m"].toIntVector();
-        return {Tensor(), once_differentiable("embed_fwd", gradient(idx, grads[0], m), grads[0].requires_grad()), Tensor(), Tensor()};
+        return {Tensor(), once_differentiable("embed_fwd", gradient(idx, grads[0], m), grads[0], {}), Tensor(), Tensor()};
     }
     static Tensor gradient(const Tensor &idx, const Tensor &grad, const std::vector<int64_t> &m)
     {
@@ -887,7 +934,7 @@ class CausalAttention : public Function<CausalAttention> {
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
         const auto saved = ctx->get_saved_variables();
-        return {once_differentiable("causal_attention", gradient(ctx, saved, grads[0]), true), Tensor(), Tensor(), Tensor()};   // qkv is an input of it
+        return {once_differentiable("causal_attention", gradient(ctx, saved, grads[0]), grads[0], {0}), Tensor(), Tensor(), Tensor()};
     }
     static Tensor gradient(AutogradContext *ctx, const variable_list &saved, const Tensor &grad)
     {
@@ -1152,6 +1199,15 @@ PyObject *py_causal_attention(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
 }
 
+// once_differentiable(grad, dy, input, input): for the functions in Python, called from their backward passes (negative: no input)
+PyObject *py_once_differentiable(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 4);
+        return THPVariable_Wrap(once_differentiable("linear", tensor_arg(a[0]), tensor_arg(a[1]), {(int)int_arg(a[2]), (int)int_arg(a[3])}));
+    });
+}
+
 // set_hooks(error class, tick)
 PyObject *py_set_hooks(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
@@ -1169,7 +1225,8 @@ PyObject *py_set_hooks(PyObject *, PyObject *const *a, Py_ssize_t n)
 PyMethodDef methods[] = {RDB_METHOD(takes_projected),   RDB_METHOD(linear_projected), RDB_METHOD(linear_one_call),
                          RDB_METHOD(linear_vector),     RDB_METHOD(embed_rows),       RDB_METHOD(set_hooks),
                          RDB_METHOD(rms_norm),          RDB_METHOD(add_rms_norm),     RDB_METHOD(relu_square),
-                         RDB_METHOD(cross_entropy),     RDB_METHOD(causal_attention), {nullptr, nullptr, 0, nullptr}};
+                         RDB_METHOD(cross_entropy),     RDB_METHOD(causal_attention), RDB_METHOD(once_differentiable),
+                         {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_rdb_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -282,6 +282,14 @@ def _dense(t: Optional[Tensor]) -> Optional[Tensor]:
     return t.get_materialized() if t is not None and hasattr(t, "get_materialized") else t
 
 
+def _once_differentiable(grad: Optional[Tensor], dy: Tensor, *inputs: int) -> Optional[Tensor]:
+    """A first derivative that a function's backward pass computed without a graph.  Under ``create_graph`` going through it again raises,
+    where dy or one of the function's tensor ``inputs`` (by number) has a gradient to come: as it is it would pass for a constant."""
+    if grad is None or not torch.is_grad_enabled() or torch.compiler.is_compiling():
+        return grad
+    return (_lib._ext or _lib.extension()).once_differentiable(grad, dy, *(inputs + (-1, -1))[:2])
+
+
 class _OneCallFunction(torch.autograd.Function):
     """``rten::linear_fwd`` and its registered backward in Python, without the operator wrappers: for the few requests the
     extension module does not take: a bias that is a pseudorandom tensor of another form than a layer's, and tensors under a
@@ -291,15 +299,24 @@ class _OneCallFunction(torch.autograd.Function):
     def forward(ctx, x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, bias):
         ctx.save_for_backward(x, coefs, scale_bias)
         ctx.meta = (in_features, out_features, stride_o, stride_i, seed)
-        ctx.bias_dtype = None if bias is None else bias.dtype
+        ctx.bias_dtype, ctx.has_scale = None if bias is None else bias.dtype, scale_bias is not None
         return hip.linear_fwd(x, coefs, in_features, out_features, stride_o, stride_i, seed, scale_bias, _dense(bias))
 
     @staticmethod
     def backward(ctx, dy):
+        dx, dcoefs, dsb = _OneCallFunction._gradients(ctx, dy)
+        dx = _once_differentiable(dx, dy, 1, 2 if ctx.has_scale else -1)
+        dcoefs, dsb = _once_differentiable(dcoefs, dy, 0), _once_differentiable(dsb, dy, 0)
+        dbias = dy.sum(0).to(ctx.bias_dtype) if ctx.bias_dtype is not None and ctx.needs_input_grad[8] else None
+        return dx, dcoefs, None, None, None, None, None, dsb, dbias
+
+    @staticmethod
+    @torch.no_grad()
+    def _gradients(ctx, dy):
         x, coefs, scale_bias = ctx.saved_tensors
         in_f, out_f, sO, sI, seed = ctx.meta
         dy = dy.contiguous()
-        dx = dcoefs = dsb = dbias = None
+        dx = dcoefs = dsb = None
         want_sb = scale_bias is not None and ctx.needs_input_grad[7]
         if ctx.needs_input_grad[0] and want_sb and sO == in_f and sI == 1:
             # the random-bias product dy.R that dx needs anyway also gives the gradient of the bias's scale (reduced against x in
@@ -315,9 +332,7 @@ class _OneCallFunction(torch.autograd.Function):
             dcoefs = dc.to(coefs.dtype)
             if want_sb:
                 dsb = ds.to(scale_bias.dtype)
-        if ctx.bias_dtype is not None and ctx.needs_input_grad[8]:
-            dbias = dy.sum(0).to(ctx.bias_dtype)
-        return dx, dcoefs, None, None, None, None, None, dsb, dbias
+        return dx, dcoefs, dsb
 
 
 class _ProjectedFunction(torch.autograd.Function):
@@ -342,17 +357,26 @@ class _ProjectedFunction(torch.autograd.Function):
         else:
             ctx.save_for_backward(state, coefs)
         ctx.meta = (in_features, out_features, seed)
-        ctx.bias_dtype = None if bias is None else bias.dtype
+        ctx.bias_dtype, ctx.has_scale = None if bias is None else bias.dtype, scale_bias is not None
         return y
 
     @staticmethod
     def backward(ctx, dy):
+        dx, dcoefs, dsb = _ProjectedFunction._gradients(ctx, dy)
+        dx = _once_differentiable(dx, dy, 1, -1 if not ctx.has_scale else 2 if ctx.bias_dtype is None else 3)
+        dcoefs, dsb = _once_differentiable(dcoefs, dy, 0), _once_differentiable(dsb, dy, 0)
+        dbias = dy.sum(0).to(ctx.bias_dtype) if ctx.bias_dtype is not None and ctx.needs_input_grad[5] else None
+        return dx, dcoefs, None, None, None, dbias, dsb
+
+    @staticmethod
+    @torch.no_grad()
+    def _gradients(ctx, dy):
         state, coefs = ctx.saved_tensors[:2]
         scale_bias, x = ctx.saved_tensors[2:] if len(ctx.saved_tensors) == 4 else (None, None)
         in_f, out_f, seed = ctx.meta
         if dy.stride(-1) != 1 or dy.stride(0) < dy.shape[1] or dy.stride(0) % 8 or dy.data_ptr() % 16:
             dy = dy.contiguous()   # the kernels read rows with a leading dimension; anything else is copied
-        dx = dcoefs = dbias = dsb = None
+        dx = dcoefs = dsb = None
         direct = not _tracing()
         want_sb = scale_bias is not None and ctx.needs_input_grad[6]
         want_dx = ctx.needs_input_grad[0] or want_sb   # the gradient of the scale comes out of the random-bias share of dx
@@ -376,11 +400,7 @@ class _ProjectedFunction(torch.autograd.Function):
             ds = hip.linear_rbias_bwd_(dx, dy, x, scale_bias, in_f, out_f, seed, want_scale_bias_grad=want_sb)
             if want_sb:
                 dsb = ds.to(scale_bias.dtype)
-        if not ctx.needs_input_grad[0]:
-            dx = None
-        if ctx.bias_dtype is not None and ctx.needs_input_grad[5]:
-            dbias = dy.sum(0).to(ctx.bias_dtype)
-        return dx, dcoefs, None, None, None, dbias, dsb
+        return dx if ctx.needs_input_grad[0] else None, dcoefs, dsb
 
 
 def _coef_form(t) -> Optional[tuple]:

@@ -212,6 +212,64 @@ def test_second_derivatives_that_do_not_exist_raise():
         first.float().sum().backward()
 
 
+@pytest.mark.parametrize("python", [False, True])
+@pytest.mark.parametrize("form", [f for f in FORMS if not f.startswith("vector")])
+def test_second_derivatives_of_a_matrix_layer_raise(form, python, monkeypatch):
+    """Its first derivatives are there under create_graph; going through them raises where they depend on something (alone, and between
+    operators that have second derivatives), and is refused as for any constant where they do not.  The bias's is linear in dy."""
+    from randumb_amd import ops
+
+    if python:   # the functions in Python, which the extension module leaves some requests to
+        monkeypatch.setattr(ops, "_bias_form", lambda bias, out_features: None)
+    layer, x = _layer(form)
+    wanted = [x, layer.weight_coef, layer.bias_coef] + ([layer.weight_scale_bias] if form.startswith("random") else [])
+    dy = torch.randn(x.shape[0], layer.out_features, device="cuda").to(x.dtype)
+    ref = torch.autograd.grad(layer(x), wanted, dy)
+    if python and form == "one_call_fp32":   # a layer takes one call here; that function's name is the module's otherwise
+        assert type(layer(x).grad_fn).__name__ == "_OneCallFunctionBackward"
+    w = dy.clone().requires_grad_()
+    for gradient in (dy, w):
+        first = torch.autograd.grad(layer(x), wanted, gradient, create_graph=True)
+        for i, (got, want) in enumerate(zip(first, ref)):
+            assert torch.linalg.vector_norm((got - want).double()) <= (1e-6 if x.dtype == torch.float32 else 1e-2) * torch.linalg.vector_norm(want.double())
+            if i != 2:
+                with pytest.raises(RuntimeError, match="second derivative"):
+                    torch.autograd.grad(got.float().square().sum(), [layer.weight_coef] if i == 0 else [x], allow_unused=True)
+    if python:   # a bias's gradient goes through the materialise operators there
+        with pytest.raises(RuntimeError, match="no autograd formula"):
+            torch.autograd.grad(first[2].sum(), w)
+    else:        # d (sum of the bias's gradient) / dy: the values of a bias with coefficients 1, for every token
+        (got,) = torch.autograd.grad(first[2].double().sum(), w)
+        want = layer.bias.get_noise_matrix().double().sum(1)
+        assert got.shape == w.shape and torch.linalg.vector_norm(got.double() - want) <= 1e-2 * torch.linalg.vector_norm(want) * x.shape[0] ** 0.5
+    # between operators with second derivatives nothing is dropped
+    s = x.detach().clone().requires_grad_()
+    (g,) = torch.autograd.grad((layer(s.square()).float() ** 2).sum(), s, create_graph=True)
+    with pytest.raises(RuntimeError, match="second derivative"):
+        torch.autograd.grad(g.float().sum(), s)
+    # nothing to come: constants, as they were
+    layer.requires_grad_(False)
+    (g,) = torch.autograd.grad(layer(x), x, dy, create_graph=True)
+    assert not g.requires_grad and torch.equal(g, ref[0])
+    layer.weight_coef.requires_grad_(True)
+    (g,) = torch.autograd.grad(layer(x.detach()), layer.weight_coef, dy, create_graph=True)
+    assert not g.requires_grad and torch.linalg.vector_norm((g - ref[1]).double()) <= 1e-2 * torch.linalg.vector_norm(ref[1].double())
+
+
+def test_a_missing_second_derivative_is_not_dropped_from_a_sum():
+    """Asked for one input by name, beside another way to it."""
+    e = SillyEmbedding(50, 24, listgen([16]), listgen([3]), device="cuda")
+    w = torch.randn(2, 24, device="cuda", requires_grad=True)
+    (first,) = torch.autograd.grad(e(torch.tensor([1, 5], device="cuda")), e.weight_coef, w, create_graph=True)
+    with pytest.raises(RuntimeError, match="second derivative"):
+        torch.autograd.grad(first.sum() + w.sum(), w)
+    qkv = torch.randn(1, 8, 192, device="cuda").bfloat16().requires_grad_()
+    y = _lib.extension().causal_attention(qkv, torch.ones(32, device="cuda"), 1, 1e-6)
+    (first,) = torch.autograd.grad(y, qkv, torch.ones_like(y), create_graph=True)
+    with pytest.raises(RuntimeError, match="second derivative"):
+        torch.autograd.grad(first.float().sum() + qkv.float().square().sum(), qkv)
+
+
 # ------------------------------------------------------------------------------------------------ slices of very wide matrices
 @pytest.mark.parametrize("sliced", ["x", "dy"])
 @pytest.mark.parametrize("form", ["projected_bf16", "projected_fp32", "random_bias_bf16", "kept_bf16"])

@@ -693,12 +693,14 @@ class VectorLinear : public Function<VectorLinear> {
     }
 };
 
-// Gradient of f(inputs...) with a graph of its own (create_graph), by f's stock operators.  Inputs without a gradient to come: undefined
-template <typename F> variable_list stock_gradient(F f, const variable_list &inputs, const variable_list &grads)
+// Gradient of f(inputs...) with a graph of its own (create_graph), by f's stock operators.  Inputs without a gradient to come: undefined.
+// f takes views of the inputs: a gradient taken at an input itself runs the hooks on it, and they run on the whole of its gradient
+// in the pass that this is part of.
+template <typename F> variable_list stock_gradient(F f, variable_list inputs, const variable_list &grads)
 {
     variable_list wanted;
-    for (const Tensor &t : inputs)
-        if (t.requires_grad()) wanted.push_back(t);
+    for (Tensor &t : inputs)
+        if (t.requires_grad()) wanted.push_back(t = t.alias());
     variable_list out(inputs.size());
     if (wanted.empty()) return out;
     const variable_list got = torch::autograd::grad(f(inputs), wanted, grads, true, true, true);

@@ -197,6 +197,34 @@ def test_second_derivatives_of_a_blocks_operators(op, strided):
         assert a.shape == b.shape and torch.linalg.vector_norm((a - b).double()) <= 1e-2 * torch.linalg.vector_norm(b.double())
 
 
+@pytest.mark.parametrize("leaf", [False, True])
+@pytest.mark.parametrize("op", ["rms_norm", "add_rms_norm", "relu_square", "cross_entropy"])
+def test_hooks_on_an_operators_input_run_once(op, leaf):
+    """Under create_graph as without it, on the whole of the input's gradient (it is used twice)."""
+    ext, eps = _lib.extension(), torch.finfo(torch.float32).eps
+    x = torch.randn(40, 64, device="cuda").bfloat16().requires_grad_()
+    t = torch.randint(0, 64, (40,), device="cuda")
+
+    def run(create):
+        seen = []
+        u = x if leaf else x * 1.0
+        handle = u.register_hook(lambda g: seen.append(g.detach().clone()))
+        if op == "add_rms_norm":
+            s, y = ext.add_rms_norm(u, u.detach(), eps)
+            s.register_hook(lambda g: seen.append(g.detach().clone()))
+            y = y + s
+        else:
+            y = {"rms_norm": lambda: ext.rms_norm(u, eps), "relu_square": lambda: ext.relu_square(u), "cross_entropy": lambda: ext.cross_entropy(u, t, -100)}[op]()
+        (g,) = torch.autograd.grad(y.float().sum() + (u.float() * 3.0).sum(), x, create_graph=create)
+        handle.remove()
+        return seen, g.detach()
+
+    (plain, g0), (graph, g1) = run(False), run(True)
+    assert len(plain) == len(graph) == (2 if op == "add_rms_norm" else 1)
+    for a, b in zip(plain + [g0], graph + [g1]):
+        assert torch.linalg.vector_norm((a - b).double()) <= 1e-2 * torch.linalg.vector_norm(a.double())
+
+
 def test_second_derivatives_that_do_not_exist_raise():
     e = SillyEmbedding(50, 24, listgen([16]), listgen([3]), device="cuda")
     w = torch.randn(2, 24, device="cuda", requires_grad=True)

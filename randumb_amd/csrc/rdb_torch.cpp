@@ -566,12 +566,7 @@ class CoefGrads : public Function<CoefGrads> {
         const auto g = coef_grads(dvalues, k, seed, true, want_scale);
         return want_scale ? variable_list{g.first, g.second} : variable_list{g.first};
     }
-    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
-    {
-        const at::AutoGradMode no_grad(false);
-        const Tensor v = coef_values(grads[0], grads.size() > 1 ? OptTensor(grads[1]) : OptTensor(), ctx->saved_data["n"].toInt(), ctx->saved_data["seed"].toInt());
-        return {v.to((at::ScalarType)ctx->saved_data["dtype"].toInt()).view(ctx->saved_data["sizes"].toIntVector()), Tensor(), Tensor(), Tensor()};
-    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads);   // by CoefValues
 };
 // The values themselves, differentiable in coef and scale.
 class CoefValues : public Function<CoefValues> {
@@ -588,6 +583,12 @@ class CoefValues : public Function<CoefValues> {
         return {g[0].to((at::ScalarType)m[2]), m[3] >= 0 ? g[1].to((at::ScalarType)m[3]) : Tensor(), Tensor(), Tensor()};
     }
 };
+
+variable_list CoefGrads::backward(AutogradContext *ctx, const variable_list &grads)
+{
+    const Tensor v = CoefValues::apply(grads[0], grads.size() > 1 ? OptTensor(grads[1]) : OptTensor(), ctx->saved_data["n"].toInt(), ctx->saved_data["seed"].toInt());
+    return {v.to((at::ScalarType)ctx->saved_data["dtype"].toInt()).view(ctx->saved_data["sizes"].toIntVector()), Tensor(), Tensor(), Tensor()};
+}
 
 std::pair<Tensor, Tensor> bias_grads_with_graph(const Tensor &dy, const std::vector<int64_t> &m)
 {

@@ -284,6 +284,27 @@ def test_second_derivatives_of_a_matrix_layer_raise(form, python, monkeypatch):
     assert not g.requires_grad and torch.linalg.vector_norm((g - ref[1]).double()) <= 1e-2 * torch.linalg.vector_norm(ref[1].double())
 
 
+@pytest.mark.parametrize("rt_bias", [False, True])
+def test_third_derivatives_of_a_vector_layer(rt_bias):
+    """The gradient of the coefficients, N^T vec(w^T x), is linear in w: the third derivatives of the sum of its fourth powers against a
+    dense matrix's."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    layer = SillyLinear(12, 9, [8, 8], [3, 4], device="cuda", bias=False, rt_bias=rt_bias)
+    x, w, u = (torch.randn(7, n, device="cuda", generator=g).requires_grad_() for n in (12, 9, 9))
+    N = layer.weight.get_noise_matrix().double()
+
+    def third(first, w, u):
+        (second,) = torch.autograd.grad((first ** 4).sum(), w, create_graph=True)
+        return torch.autograd.grad((second * u).square().sum(), [w, u])
+
+    (first,) = torch.autograd.grad(layer(x), layer.weight_coef, w, create_graph=True)
+    got = third(first, w, u)
+    w64, u64 = w.detach().double().requires_grad_(), u.detach().double().requires_grad_()
+    want = third(N.t() @ (w64.t() @ x.detach().double()).flatten(), w64, u64)
+    for a, b in zip(got, want):
+        assert torch.linalg.vector_norm(a.double() - b) <= 1e-4 * torch.linalg.vector_norm(b)
+
+
 def test_a_missing_second_derivative_is_not_dropped_from_a_sum():
     """Asked for one input by name, beside another way to it."""
     e = SillyEmbedding(50, 24, listgen([16]), listgen([3]), device="cuda")

@@ -80,7 +80,7 @@ __device__ __forceinline__ Split8 few_split8(const f32x8 &v)
     return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
 }
 // The same with the parts cut off and not rounded, all of one sign: no two of a product's terms overflow to different sides.  What is
-// left out of a product of two such splits is up to 2^-21 of it and of its sign, so only sums that came out not finite are done with it.
+// left out of a product of two such splits is up to 2^-21 of it and of its sign, so only sums that came out not finite are taken from it.
 __device__ __forceinline__ Split8 few_split8_any(const f32x8 &v)
 {
     constexpr float top = 3.40282346638528859812e38f;
@@ -396,12 +396,22 @@ template <typename E, int KS, int TT, bool MANY> __device__ __forceinline__ void
         }
     };
     product(std::false_type{});
+    f32x4 sum[TT];
     float zero = 0.0f;   // stays so as long as every sum is finite
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt)
+    for (int tt = 0; tt < TT; ++tt) {
+        sum[tt] = acc[tt] + low[tt];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) zero = tt * 16 + r < T ? fmaf(acc[tt][j] + low[tt][j], 0.0f, zero) : zero;
-    if (__any(zero != 0.0f)) product(std::true_type{});
+        for (int j = 0; j < 4; ++j) zero = tt * 16 + r < T ? fmaf(sum[tt][j], 0.0f, zero) : zero;
+    }
+    if (__any(zero != 0.0f)) {   // once more, for the sums that are not finite: the others stay as they would be without these beside them
+        product(std::true_type{});
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (sum[tt][j] * 0.0f != 0.0f) sum[tt][j] = acc[tt][j] + low[tt][j];
+    }
     // result element j of lane (r, g): output feature o0 + 4 g + j, token r
     const int o = o0 + g * 4;
     float bv[4];
@@ -413,7 +423,7 @@ template <typename E, int KS, int TT, bool MANY> __device__ __forceinline__ void
         if (t >= T || o >= p.out_f) continue;
         float v[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = acc[tt][j] + low[tt][j] + bv[j];
+        for (int j = 0; j < 4; ++j) v[j] = sum[tt][j] + bv[j];
         E *const dst = y + (int64_t)t * p.ldy + o;
         if (p.y_vec) {   // out_f is a multiple of 4
             if constexpr (sizeof(E) == 2) *reinterpret_cast<uint2 *>(dst) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));

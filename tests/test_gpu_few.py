@@ -76,6 +76,25 @@ def test_not_finite(k, dtype):
     assert bool(((y - want).abs() <= bound)[ok].all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,in_f,out_f,k", [(5, 96, 70, 2), (16, 512, 64, 16), (40, 300, 130, 33), (33, 2048, 5000, 64)])
+def test_a_value_that_is_not_finite_leaves_its_neighbours_alone(T, in_f, out_f, k, dtype):
+    """Other tokens of the call and other output features: bit for bit what they are without it."""
+    x, c, b, _ = _case(T, in_f, out_f, k, dtype)
+    call = lambda x, c: hip.linear_fwd(x, c, in_f, out_f, in_f, 1, 5, bias=b)
+    want = call(x, c)
+    t, o = T - 2, out_f - 3
+    for bad in (float("inf"), float("nan"), 3.0e38):
+        spoiled = x.clone()
+        spoiled[t, in_f // 2] = bad
+        got = call(spoiled, c)
+        assert torch.equal(got[torch.arange(T) != t], want[torch.arange(T) != t])
+        spoiled = c.clone()
+        spoiled[o, k - 1] = bad
+        got = call(x, spoiled)
+        assert torch.equal(got[:, torch.arange(out_f) != o], want[:, torch.arange(out_f) != o])
+
+
 def test_recorded_launches():
     """Both forms recorded into one graph and replayed on changing inputs, with eager calls in between."""
     shapes = [(5, 1001, 999, 99), (100, 264, 352, 64), (16, 4096, 4096, 256), (40, 8192, 512, 512)]   # one launch (one group of tokens, four), two, three

@@ -72,7 +72,7 @@ __device__ __forceinline__ void fg_split3(float v0, float v1, uint32_t &h, uint3
 // and not rounded: all of one sign, so that none of a product's terms overflows to the other side.  A NaN stays a NaN.  This takes two
 // v_med3 a value, 3 % of a step (2048 tokens x 768 -> 3072, k = 256, fp32: 107 -> 110 us, and 112 with a look at each stage's
 // values instead), so it is not done at first: an infinity then gives NaN wherever it is met, and a block whose sums are not all
-// finite runs its stages once more with it (104.4 us, against 103.4 without any of it in the same run).  A value that comes from
+// finite runs its stages once more with it, for those (104.4 us, against 103.4 without any of it in the same run).  A value that comes from
 // a bf16 matrix has one part, and an infinite one gives NaN where its partner's lower parts are zero: the products of bf16
 // layers do without the second run.
 __device__ __forceinline__ void fg_split3_any(float v, uint32_t &h, uint32_t &m, uint32_t &l)
@@ -398,7 +398,7 @@ __device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, 
     typedef FgBlock<BM, G, ASRC, BSRC, VEC, SPLIT, AES, BES> Block;
     typedef typename Block::PA PA;
     typedef typename Block::PB PB;
-    constexpr bool ANY16 = PA::ONE || PB::ONE;
+    constexpr bool ANY16 = PA::ONE || PB::ONE, AGAIN = SPLIT && !ANY16;   // AGAIN: sums that are not finite are looked for
     constexpr int MI = Block::MI, NI = Block::NI, STAGE = Block::STAGE, UNITS = Block::UNITS;
     const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / FG_THREADS);
     float *lds = lds_all + group * 2 * STAGE;
@@ -418,7 +418,7 @@ __device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, 
     // quarter of their waves (2048 tokens x 768 -> 3072, k = 256: step 106.5 us against 104.4); their contractions are short.
     constexpr bool APART = SPLIT && BM == 64 && G > 1 && !ANY16;
     f32x16 acc[MI][NI], low[MI][NI];
-    if (SPLIT && !ANY16 && threadIdx.x == 0) not_finite = 0;   // seen by everybody behind the first stage's barrier
+    if (AGAIN && threadIdx.x == 0) not_finite = 0;   // seen by everybody behind the first stage's barrier
     // The stage loop; for fp32 matrices once more for sums that are not finite (fg_split3).  A side that comes from a bf16 matrix has one
     // plane.
     auto stages = [&](auto finite) __attribute__((always_inline)) {
@@ -530,7 +530,7 @@ __device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, 
     };
     product(std::true_type{});
     bool again = false;
-    if (SPLIT && !ANY16) {
+    if (AGAIN) {
         float zero = 0.0f;   // stays so as long as every sum is finite
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi)
@@ -541,12 +541,10 @@ __device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, 
         if (zero != 0.0f) not_finite = 1;
         __syncthreads();   // also: the stage buffers are free
         again = __builtin_amdgcn_readfirstlane(not_finite) != 0;
-        if (again) product(std::false_type{});
     }
-    if constexpr (G > 1) {
-        const bool behind_barrier = !ANY16 && !again;
-        // unit u (registers 8 (u % 2) .. of tile u / 2) is finished by group u * G / UNITS; the others hand theirs over
-        if (!behind_barrier) __syncthreads();   // the stage buffers are free
+    // The groups' sums: unit u (registers 8 (u % 2) .. of tile u / 2) is finished by group u * G / UNITS; the others hand theirs over.  Behind a
+    // barrier: the stage buffers are free
+    auto exchange = [&]() __attribute__((always_inline)) {
         auto slot = [&](int u, int from, int owner) { return lds_all + ((u * (G - 1) + (from < owner ? from : from - 1)) * 4 + wave) * 512 + lane; };
 #pragma unroll
         for (int u = 0; u < UNITS; ++u) {
@@ -569,6 +567,10 @@ __device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, 
                 for (int j = 0; j < 8; ++j) acc[u / 2 / NI][u / 2 % NI][(u & 1) * 8 + j] += src[j * 64];
             }
         }
+    };
+    if constexpr (G > 1) {
+        if (!AGAIN) __syncthreads();
+        exchange();
     }
     // accumulator j of lane (r, g): row 8 (j / 4) + 4 g + j % 4 of the A side, column r of the B side
     float *out = p.out + (int64_t)bz * p.split_stride;
@@ -577,14 +579,21 @@ __device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, 
     const float scale = (EPI != FG_ADD_SCALED && EPI != FG_STORE_RBIAS) ? 0.0f
                         : p.scale_bf16 ? bf16_to_f32(reinterpret_cast<const bf16_t *>(p.scale)[0]) : p.scale[0];
     float dot = 0.0f;
-    // KIND: how the results leave, where that is known outside of the loops (a branch per store costs 4 us of the fp32 step above)
+    // KIND: how the results leave, where that is known outside of the loops (a branch per store costs 4 us of the fp32 step above).
+    // Sums that are not finite come from the stages run once more (fg_split3_any), and only those: the others leave as they do without
+    // these beside them.  WHICH: all; or, from the second run, those in whose place the first one left a value that is not finite.
+    // What is added to an output is not seen there: the first run then leaves out the sums that are not finite, `bad`, for the second.
     enum { STREAM, PLAIN, NARROW, ANY };
-    auto results = [&](auto kind) __attribute__((always_inline)) {
-        constexpr int KIND = decltype(kind)::value;
+    enum { ALL, REPAIR, GOOD, BAD };
+    uint32_t bad[MI * NI / 2];
+    auto results = [&](auto kind, auto which) __attribute__((always_inline)) {
+        constexpr int KIND = decltype(kind)::value, WHICH = decltype(which)::value;
         const bool to16 = KIND == NARROW || (KIND == ANY && o16);
+        int r_ = r, g_ = g;
+        if (WHICH != ALL) asm volatile("" : "+v"(r_), "+v"(g_));   // addresses are made here and not kept in registers over the stages
 #pragma unroll
         for (int ni = 0; ni < NI; ++ni) {
-            const int n = n0 + wn * 64 + ni * 32 + r;
+            const int n = n0 + wn * 64 + ni * 32 + r_;
             if (n >= p.N) continue;
             const float bv = EPI != FG_STORE_BIAS ? 0.0f : to16 ? bf16_to_f32(reinterpret_cast<const bf16_t *>(p.bias)[n]) : p.bias[n];
 #pragma unroll
@@ -592,8 +601,9 @@ __device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, 
 #pragma unroll
                 for (int j = 0; j < 16; ++j) {
                     if (G > 1 && group != ((mi * NI + ni) * 2 + j / 8) * G / UNITS) continue;
-                    const int m = m0 + wm * (BM / 2) + mi * 32 + 8 * (j >> 2) + 4 * g + (j & 3);
+                    const int m = m0 + wm * (BM / 2) + mi * 32 + 8 * (j >> 2) + 4 * g_ + (j & 3);
                     if (m >= p.M) continue;
+                    if ((WHICH == GOOD || WHICH == BAD) && (bad[(mi * NI + ni) / 2] >> ((mi * NI + ni) % 2 * 16 + j) & 1) != (WHICH == BAD)) continue;
                     const float a = acc[mi][ni][j];
                     if (EPI == FG_DOT || (EPI == FG_ADD_SCALED && p.dotm)) {
                         const int64_t e = (int64_t)m * p.lddot + n;
@@ -601,6 +611,7 @@ __device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, 
                     }
                     if (EPI != FG_DOT) {
                         const int64_t e = (int64_t)m * p.ldo + n;
+                        if (WHICH == REPAIR && (to16 ? bf16_to_f32(out16[e]) : out[e]) * 0.0f == 0.0f) continue;
                         if (EPI == FG_STORE_RBIAS) out[e] = fmaf(scale, noise1d((uint32_t)m * p.nsR + (uint32_t)n * p.nsK, p.seed), a);
                         else if (to16) out16[e] = f32_to_bf16(EPI == FG_ADD_SCALED ? fmaf(scale, a, bf16_to_f32(out16[e])) : a + bv);
                         else if (EPI == FG_ADD_SCALED) out[e] = fmaf(scale, a, out[e]);
@@ -610,12 +621,46 @@ __device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, 
                 }
         }
     };
-    if constexpr (EPI == FG_STORE || EPI == FG_STORE_BIAS) {
-        if (o16) results(std::integral_constant<int, NARROW>{});
-        else if (p.ldo % 32 == 0) results(std::integral_constant<int, STREAM>{});   // rows of whole lines
-        else results(std::integral_constant<int, PLAIN>{});
+    typedef std::integral_constant<int, ANY> Any;
+    typedef std::integral_constant<int, ALL> All;
+    auto second_run = [&]() __attribute__((always_inline)) {
+        __syncthreads();   // the groups' sums have been read
+        product(std::false_type{});
+        if constexpr (G > 1) {
+            __syncthreads();
+            exchange();
+        }
+    };
+    if constexpr (EPI == FG_ADD_SCALED || EPI == FG_DOT) {
+        if (again) {
+#pragma unroll
+            for (int i = 0; i < MI * NI / 2; ++i) {
+                bad[i] = 0;
+#pragma unroll
+                for (int e = 0; e < 32; ++e) bad[i] |= acc[(2 * i + e / 16) / NI][(2 * i + e / 16) % NI][e % 16] * 0.0f != 0.0f ? 1u << e : 0u;
+                asm volatile("" : "+v"(bad[i]));   // a word, not 32 comparisons
+            }
+            results(Any{}, std::integral_constant<int, GOOD>{});
+        } else {
+            results(Any{}, All{});
+        }
+        if constexpr (AGAIN) {
+            if (again) {
+                second_run();
+                results(Any{}, std::integral_constant<int, BAD>{});
+            }
+        }
     } else {
-        results(std::integral_constant<int, ANY>{});
+        if constexpr (EPI == FG_STORE_RBIAS) results(Any{}, All{});
+        else if (o16) results(std::integral_constant<int, NARROW>{}, All{});
+        else if (p.ldo % 32 == 0) results(std::integral_constant<int, STREAM>{}, All{});   // rows of whole lines
+        else results(std::integral_constant<int, PLAIN>{}, All{});
+        if constexpr (AGAIN) {
+            if (again) {
+                second_run();
+                results(Any{}, std::integral_constant<int, REPAIR>{});
+            }
+        }
     }
     if (EPI == FG_DOT || (EPI == FG_ADD_SCALED && p.dotm)) {
         // lanes, then waves, in a fixed order

@@ -83,6 +83,45 @@ def test_projection_and_its_products(tokens, in_f, out_f, k):
     same_pattern(dc, dy.double().t() @ (x.double() @ N))
 
 
+# tiles of 128 and 64 rows, one group of waves and several, one range of the contraction and several, pieces that are and are not aligned; the
+# random bias's share is added to an output
+@pytest.mark.parametrize("form", ["matrix", "random_bias", "vector"])
+@pytest.mark.parametrize("tokens,in_f,out_f,k", [(600, 256, 192, 70), (2048, 768, 3072, 256), (4100, 301, 259, 83), (2000, 2001, 130, 66), (700, 2048, 2048, 512)])
+def test_finite_sums_are_what_they_are_without_others_beside_them(form, tokens, in_f, out_f, k):
+    """An infinity, a NaN or a product beyond the largest float in a row of x or in one value of dy: the other rows and columns keep
+    their bits."""
+    if form == "vector" and (k > 100 or in_f > 400):
+        k = 16
+    print(f"case beside {form} {tokens} x {in_f} -> {out_f}, k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    layer = SillyLinear(in_f, out_f, [k, k], [3, 4], device="cuda", bias=False, matrix_coef=form != "vector", rt_bias=form == "random_bias")
+    with torch.no_grad():
+        layer.weight_coef.normal_(0.0, 0.1, generator=g)
+    x, dy = torch.randn(tokens, in_f, device="cuda", generator=g), torch.randn(tokens, out_f, device="cuda", generator=g)
+
+    def run(x, dy):
+        x = x.clone().requires_grad_()
+        y = layer(x)
+        dx, dc = torch.autograd.grad(y, [x, layer.weight_coef], dy)
+        return y.detach(), dx, dc
+
+    y, dx, dc = run(x, dy)
+    row, col = tokens - 3, out_f // 2
+    rows, cols = torch.arange(tokens, device="cuda") != row, torch.arange(out_f, device="cuda") != col
+    for bad in (math.inf, math.nan, 3.0e38):
+        spoiled = x.clone()
+        spoiled[row, in_f // 3] = bad
+        got = run(spoiled, dy)
+        assert torch.equal(got[0][rows], y[rows]) and torch.equal(got[1], dx)
+        spoiled = dy.clone()
+        spoiled[row, col] = bad
+        got = run(x, spoiled)
+        assert torch.equal(got[0], y) and torch.equal(got[1][rows], dx[rows])
+        assert form == "vector" or torch.equal(got[2][cols], dc[cols])
+        if bad != 3.0e38:   # as it has to be: no value of the row is finite
+            assert not bool(got[1][row].isfinite().any())
+
+
 def test_the_largest_values_do_not_become_nan():
     """Parts of one sign: a product that overflows is an infinity of its own sign, one that does not is finite."""
     layer = SillyLinear(64, 32, [8, 8], [3, 4], device="cuda", bias=False)

@@ -24,6 +24,8 @@
 
 namespace rdb {
 
+int f32_split_mode();   // rdb_f32.hip
+
 constexpr int FEW_ROWS = 64;       // output features of an expanding block: 16 a wave
 constexpr int FEW_COEFS = 16;      // coefficients of a contracting block
 constexpr int FEW_STEPS = 4;       // steps of 32 contraction values a contracting wave hashes ahead of its products
@@ -548,6 +550,7 @@ static bool few_pays(const rdb_linear_desc *d)
 static bool few_ok(const rdb_linear_desc *d)
 {
     const bool f32 = d->act_dtype == RDB_F32 && d->coef_dtype == RDB_F32, b16 = d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16;
+    if (!f32_split_mode() && !(b16 && d->in_f % 8 == 0 && d->out_f % 8 == 0 && d->k % 8 == 0)) return false;   // fp32 products are asked for (rdb_set_f32_split)
     return (f32 || b16) && d->algo == RDB_ALGO_AUTO && d->coef_rows != 0 && d->k > 0 && d->k <= FEW_K && d->tokens > 0 && d->in_f > 0 &&
            d->out_f > 0 && d->in_f < (1 << 20) && d->out_f < (1 << 24) && few_pays(d) && d->k * (d->in_f + d->out_f) < 16 * d->in_f * d->out_f;
 }

@@ -95,6 +95,22 @@ def test_a_value_that_is_not_finite_leaves_its_neighbours_alone(T, in_f, out_f, 
         assert torch.equal(got[:, torch.arange(out_f) != o], want[:, torch.arange(out_f) != o])
 
 
+@pytest.mark.parametrize("T,in_f,out_f,k", [(20, 1000, 520, 100), (200, 512, 512, 128), (3, 4096, 300, 16), (500, 700, 333, 40)])
+def test_fp32_products_where_they_are_asked_for(T, in_f, out_f, k):
+    """rdb_set_f32_split(0): a forward of few tokens in fp32 leaves the split products too, for the kernels that FACTORED names."""
+    x, c, b, N = _case(T, in_f, out_f, k, torch.float32)
+    call = lambda algo: hip.linear_fwd(x, c, in_f, out_f, in_f, 1, 5, bias=b, algo=algo)
+    split = call(_lib.RDB_ALGO_AUTO)
+    before = hip.set_f32_split(0)
+    try:
+        plain = call(_lib.RDB_ALGO_AUTO)
+        assert torch.equal(plain, call(_lib.RDB_ALGO_FACTORED)) or k <= 64   # k <= 64: AUTO chooses between two kernels, FACTORED does not
+    finally:
+        hip.set_f32_split(before)
+    assert not torch.equal(plain, split) and _rel(plain, (x.double() @ N) @ c.double().t() + b.double()) < 1e-5
+    assert torch.equal(call(_lib.RDB_ALGO_AUTO), split)
+
+
 def test_recorded_launches():
     """Both forms recorded into one graph and replayed on changing inputs, with eager calls in between."""
     shapes = [(5, 1001, 999, 99), (100, 264, 352, 64), (16, 4096, 4096, 256), (40, 8192, 512, 512)]   # one launch (one group of tokens, four), two, three

@@ -226,6 +226,33 @@ def test_f32_split_switch_without_a_gpu():
     assert L.rdb_set_f32_split(first) == first
 
 
+def test_f32_split_switch_reaches_few_token_forwards():
+    """The scratch of the kernels for few tokens, which split their operands, is asked for only where they would run: with fp32 products
+    asked for neither for fp32 nor for bf16 with sizes that are not multiples of 8."""
+    import ctypes
+
+    import torch
+
+    from randumb_amd import _lib, hip
+
+    L = _lib.load()
+
+    def needs(T, in_f, out_f, k, dtype):
+        d = hip._desc(T, in_f, out_f, torch.empty(out_f, k, dtype=dtype, device="meta"), in_f, 1, 5, dtype, _lib.RDB_ALGO_AUTO)
+        sizes = []
+        for mode in (1, 0):
+            before = L.rdb_set_f32_split(mode)
+            sizes.append(L.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_FWD, ctypes.byref(d)))
+            L.rdb_set_f32_split(before)
+        return sizes
+
+    for dtype in (torch.float32, torch.bfloat16):
+        split, plain = needs(20, 1001, 999, 99, dtype)
+        assert 0 < plain < split
+    split, plain = needs(20, 1000, 1000, 96, torch.bfloat16)
+    assert split == plain
+
+
 def test_argument_errors_come_back_as_codes_without_a_gpu():
     from randumb_amd import _lib
 

@@ -55,10 +55,13 @@ constexpr int COEF_CHUNK = 2048;
 // term by term.  Without it, and with MAT_UNROLL terms a turn of the loop (still one after the other), a term takes 17 vector instructions
 // instead of 19: 768 x 3072 elements, k = 256: 219 -> 205 us, and the pass of that layer, 1024 tokens, 538 -> 520; 4096 rows of a 50304 x
 // 768 table, forward and backward, 525 -> 522 (one term a turn: 540).  The round constants stay literals: in scalar or vector registers the
-// same instructions take 2 to 6 % longer.  What is left of a chunk goes by fours and twos: 618 x 2480 elements, k = 23, 21.2 -> 20.9 us (with the
-// factor term by term and without the look at the coefficients 19.9: at so few terms the look is not paid back).
+// same instructions take 2 to 6 % longer.  What is left of a chunk goes by fours and twos.  The look at the coefficients costs a launch about
+// a microsecond, which up to MAT_SHORT terms are not paid back: those get the factor term by term.  768 x 3072 elements, term by term
+// and otherwise: k = 8 11.8 and 13.9 us, 23 22.9 and 24.5, 48 41.2 and 42.1, 64 52.9 and 53.6, 96 76.6 and 76.5, 256 194 and 190; 300 x 800
+// elements: 48 8.5 both, 64 9.1 and 8.7.
 constexpr float MAT_LARGE = 3.777893186295716e22f;   // 2^75
 constexpr int MAT_UNROLL = 8;
+constexpr int MAT_SHORT = 48;
 
 struct MatVecParams {
     float *out;
@@ -71,8 +74,8 @@ struct MatVecParams {
 
 // LANES > 1: that many neighbouring lanes share an element, lane l its terms l, l + LANES, .. (then added up across the lanes, nearest
 // first): with few elements the chip is not full, and the chain's length is what a launch takes (3072 elements, k = 256: 16.5 ->
-// 4 us).
-template <bool GATHER, int LANES> __global__ __launch_bounds__(NT) void materialize_vec_kernel(MatVecParams p)
+// 4 us).  SHORT: at most MAT_SHORT terms.
+template <bool GATHER, int LANES, bool SHORT> __global__ __launch_bounds__(NT) void materialize_vec_kernel(MatVecParams p)
 {
     __shared__ __align__(16) float cs[COEF_CHUNK];
     const int64_t n = ((int64_t)blockIdx.x * NT + threadIdx.x) / LANES;
@@ -94,7 +97,8 @@ template <bool GATHER, int LANES> __global__ __launch_bounds__(NT) void material
             cs[j] = c;
             large |= !(fabsf(c) < MAT_LARGE);
         }
-        if (__syncthreads_or(large)) {
+        if (SHORT) __syncthreads();
+        if (SHORT || __syncthreads_or(large)) {
             if (live)
                 for (int j = part; j < cnt; j += LANES) {
                     acc = fmaf(sq5_unit(sq5_tail_apart(first)), cs[j], acc);
@@ -507,8 +511,13 @@ static int launch_materialize_vec(float *out, const void *coef, int coef_dtype, 
     const unsigned blocks = (unsigned)cdiv(Nw * lanes, NT);
     auto launch = [&](auto lanes_) {
         constexpr int L = decltype(lanes_)::value;
-        if (idx) materialize_vec_kernel<true, L><<<blocks, NT, 0, s>>>(p);
-        else materialize_vec_kernel<false, L><<<blocks, NT, 0, s>>>(p);
+        auto run = [&](auto short_) {
+            constexpr bool SHORT = decltype(short_)::value;
+            if (idx) materialize_vec_kernel<true, L, SHORT><<<blocks, NT, 0, s>>>(p);
+            else materialize_vec_kernel<false, L, SHORT><<<blocks, NT, 0, s>>>(p);
+        };
+        if (k <= MAT_SHORT) run(std::true_type{});
+        else run(std::false_type{});
     };
     if (lanes == 16) launch(std::integral_constant<int, 16>{});
     else if (lanes == 4) launch(std::integral_constant<int, 4>{});

@@ -109,3 +109,15 @@ def test_terms_with_and_without_their_common_factor(hip, n, k):
             assert rel(got, noise * 3.0e37) < 1e-6
     c[k - 1] = float("inf")
     assert not bool(torch.isfinite(values(c)).any())
+
+
+@pytest.mark.parametrize("n,k", [(3000, 47), (3000, 48), (70001, 48), (3000, 49), (70001, 49), (300, 49), (70001, 55)])
+def test_few_terms_and_more(hip, n, k):
+    """Up to 48 terms have the factor applied term by term, more do not: the same sums on either side of the line."""
+    test_terms_with_and_without_their_common_factor(hip, n, k)
+    g = torch.Generator(device="cuda").manual_seed(n * k)
+    c = torch.randn(k, generator=g, device="cuda")
+    noise = hip.sq5_fill_2d(n, k, 11).double()
+    got = hip.materialize_fwd(c, (n,), (1,), 11, None, False)
+    # k fp32 multiply-adds one after the other, each rounded by at most 2^-24 of the running sum
+    assert float((got.double() - noise @ c.double()).abs().max()) <= k * 2.0**-24 * float((noise.abs() @ c.double().abs()).max())

@@ -398,21 +398,24 @@ template <typename E, int KS, int TT, bool MANY> __device__ __forceinline__ void
         }
     };
     product(std::false_type{});
-    f32x4 sum[TT];
     float zero = 0.0f;   // stays so as long as every sum is finite
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-        sum[tt] = acc[tt] + low[tt];
+    for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) zero = tt * 16 + r < T ? fmaf(sum[tt][j], 0.0f, zero) : zero;
-    }
+        for (int j = 0; j < 4; ++j) zero = tt * 16 + r < T ? fmaf(acc[tt][j] + low[tt][j], 0.0f, zero) : zero;
     if (__any(zero != 0.0f)) {   // once more, for the sums that are not finite: the others stay as they would be without these beside them
+        f32x4 sum[TT];
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) sum[tt] = acc[tt] + low[tt];
         product(std::true_type{});
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                if (sum[tt][j] * 0.0f != 0.0f) sum[tt][j] = acc[tt][j] + low[tt][j];
+                if (sum[tt][j] * 0.0f == 0.0f) {
+                    acc[tt][j] = sum[tt][j];
+                    low[tt][j] = -0.0f;
+                }
     }
     // result element j of lane (r, g): output feature o0 + 4 g + j, token r
     const int o = o0 + g * 4;
@@ -425,7 +428,7 @@ template <typename E, int KS, int TT, bool MANY> __device__ __forceinline__ void
         if (t >= T || o >= p.out_f) continue;
         float v[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = sum[tt][j] + bv[j];
+        for (int j = 0; j < 4; ++j) v[j] = acc[tt][j] + low[tt][j] + bv[j];
         E *const dst = y + (int64_t)t * p.ldy + o;
         if (p.y_vec) {   // out_f is a multiple of 4
             if constexpr (sizeof(E) == 2) *reinterpret_cast<uint2 *>(dst) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));

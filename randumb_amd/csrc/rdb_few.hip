@@ -483,10 +483,12 @@ template <typename E, int KS, int TC, int TE> __global__ __launch_bounds__(256, 
 // sum: beyond 200 KB of partial sums for a block they are added up once, by a launch of its own, and not by every expanding block
 // (48 to a block, 32 tokens x 4096 -> 11008, k = 256: 15.6 -> 14.9 us; 16 tokens, 131 KB: 11.5, and 12.7 with it).
 // one: a single launch where the expanding blocks are few and the partial sums of each small; tags and reads that go around L2 cost many
-// blocks more than a launch does (16 x 4096 -> 11008, k = 256: two launches 11.5, one 13.5), but a program's host takes 10.7 us to issue two.
-// us of a program's call, two launches -> one: 5 x 1001 -> 999, k = 99: 9.2 -> 7.5 (library calls); 100 x 264 -> 352, k = 64, 42 blocks: 11.0 ->
-// 8.6; 32 x 1024 -> 2048, k = 128, 64 blocks of 64 KB: 10.8 -> 9.2; 4 x 2048 -> 10000, k = 32, 157 blocks: 10.8 -> 9.1; 64 x 768 -> 2048, k = 64, 128
-// blocks: 10.9 -> 10.0; 256 x 512 -> 640, k = 128, fp32, 160 blocks of 32 KB: 11.2 -> 11.7.
+// blocks more than a launch does (16 x 4096 -> 11008, k = 256: two launches 11.5, one 13.5), but a program's host takes 9.0 to 11.7 us (by
+// the box and by what the program does between calls) to issue two, and those calls then take that.  us of a call in one launch, which
+// the host does not hold up: 5 x 1001 -> 999, k = 99: 7.8; 48 x 768 -> 768, k = 64: 8.3; 100 x 264 -> 352, k = 64: 8.7; 32 x 1024 -> 2048,
+// k = 128, 64 blocks of 64 KB: 9.2; 4 x 2048 -> 10000, k = 32, 157 blocks: 9.0; 64 x 768 -> 2048, k = 64, 128 blocks: 9.9.  At the line the
+// two are about even, whichever the host: 256 x 512 -> 640, k = 128, 160 blocks of 32 KB and 256 tags: 10.7 in bf16 and 11.6 in fp32, two launches
+// 9.3 and 9.7 on the fastest host, 11.7 and 11.5 in a program; 224 x 512 -> 640, k = 96, 140 blocks, 168 tags, bf16: 12.2, and 9.5 or 11.3.
 struct FewPlan {
     int wave_values, chunks, ranges;
     int tile, tiles, tc, te;

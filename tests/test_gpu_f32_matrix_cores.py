@@ -163,6 +163,19 @@ def test_rows_that_end_inside_a_piece_of_four(hip, oracle, in_f, out_f, k, dtype
     assert rel_l2(dc.cpu().numpy(), want_dc) < F32_TOL
 
 
+@pytest.mark.parametrize("in_f,out_f,k", [(1, 2, 3), (2, 9, 1), (3, 5, 2), (4, 6, 5), (5, 3, 7), (17, 15, 18), (66, 131, 19), (259, 126, 65)])
+def test_rows_of_coefficients_that_end_inside_a_piece_of_four(hip, oracle, in_f, out_f, k):
+    """The same for a forward in bf16 of more tokens than rdb_few.hip takes: y = z . C^T with z in fp32 and bf16 rows of C of any length."""
+    T, seed = 531, 23
+    x, _, coef, bias = (v.bfloat16() for v in _inputs(T, in_f, out_f, k, seed))
+    wide = torch.full((T, in_f + 3), float("nan"), device="cuda", dtype=torch.bfloat16)
+    wide[:, :in_f] = x.cuda()
+    want = oracle.linear_fwd(x.float().numpy(), coef.float().numpy(), in_f, out_f, seed, bias=bias.float().numpy())
+    print(f"case f32 matrix cores edges in={in_f} out={out_f} k={k} bf16 T={T}", flush=True)
+    y = hip.linear_fwd(wide[:, :in_f], coef.cuda(), in_f, out_f, in_f, 1, seed, bias=bias.cuda())
+    assert rel_l2(y.float().cpu().numpy(), want) < 2.0**-8   # fp32 sums, rounded once
+
+
 def test_layer_level_fp32(hip, oracle):
     """SillyLinear(matrix_coef=True) in fp32 at a GPT-like slice: forward, input gradient and coefficient gradient through autograd."""
     from randumb_amd.SillyLayers import SillyLinear

@@ -77,6 +77,12 @@ def test_few_token_forward_and_dx_on_the_matrix_cores(T, in_f, out_f, k):
     assert rc == 0 and _rel(y, x.double() @ W.t()) < 5e-6
 
 
+# the forward of up to 512 tokens is rdb_few.hip's: the same rule above that, with products of either kind the faster ones
+@pytest.mark.parametrize("T,in_f,out_f,k", [(513, 128, 256, 64), (700, 785, 257, 33), (520, 2000, 100, 16), (600, 1030, 130, 8)])
+def test_forward_and_dx_of_more_than_a_few_tokens(T, in_f, out_f, k):
+    test_few_token_forward_and_dx_on_the_matrix_cores(T, in_f, out_f, k)
+
+
 # every kind of block the pair of products in one launch is planned for (128 rows with one group and with two, 64 rows with two), with
 # one and with several ranges on either side, whole and ragged tiles, pieces of four that are and are not aligned
 @pytest.mark.parametrize("T,in_f,out_f,k,dtype", [(131, 259, 129, 65, torch.float32), (131, 259, 129, 65, torch.bfloat16), (2048, 768, 3072, 256, torch.float32),

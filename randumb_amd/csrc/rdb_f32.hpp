@@ -720,8 +720,10 @@ inline FgPlan fg_room(int64_t M, int64_t N, int64_t K, int num_cus, int64_t min_
 // file's kinds, [258 .. 7520] x [100 .. 7520] over [100 .. 7520], some 380 plans; what it picks is within 1 % of the best of
 // them on average, 3 % at most): a stage of a group takes `chain` us when it has the compute unit to itself, the groups that
 // share a unit take `unit` us of its throughput each, a launch `base` us and every further round of blocks 2.6; outputs leave at 4.8 TB/s; adding ranges up is one more
-// launch, whose 14 TB/s say that the partial matrices come back out of the caches.  Blocks that run on a unit at a time: what
-// registers and LDS leave room for.
+// launch, whose 14 TB/s say that the partial matrices come back out of the caches.  `resident`, the groups that take turns on a unit's
+// time, was fitted with the others and is not what registers and LDS leave room for.  The products measured had fp32 matrices; a
+// side that comes from a bf16 matrix takes less LDS and fewer registers (four to seven blocks of 256 threads fit a unit), and hashing
+// is not told apart: for those the constants are what they are for fp32.
 struct FgKind {
     int bm, groups, resident;
     double chain, unit, base;
@@ -761,7 +763,8 @@ inline FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int max_rang
 // Two products side by side in one launch, blocks of one kind (rdb_f32_pair.hip).  The same model with constants of its own, fitted to
 // 14 layers of 256 to 8000 tokens ([300 .. 3001] -> [256 .. 8192], k 40 to 700), some 100 plans each: what it picks is within 5 % of
 // the backward pass of the best of them (1 % on average).  chain, unit: as above; a unit's blocks are of both products, so the mean of
-// their stages counts; out, sum: us per MB of partial matrices written, and read back; resident: bf16 matrices take less LDS.
+// their stages counts; out, sum: us per MB of partial matrices written, and read back; resident: fitted as the others are (of 128 rows
+// and two groups one block fits a unit whatever the matrices, 132 registers and 512 threads in bf16; two say that rounds cost less).
 struct FgPairPlan {
     int bm, groups, ranges[2];
 };

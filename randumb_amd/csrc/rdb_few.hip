@@ -9,7 +9,7 @@
 // launch, the two kinds of block are two launches of the same kernel.
 // us per call, three launches on the vector ALU (or the kernels for many tokens) -> here: 16 tokens x 4096 -> 11008, k = 256, bf16 14.5 ->
 // 11.5; 1 x 7512 -> 2376, k = 512, bf16 34.6 -> 14.0; 5 x 1001 -> 999, k = 99, bf16 17.1 -> 7.5; 22 x 264 -> 352, k = 64, fp32 17.7 -> 8.6;
-// 1 x 4096 -> 4096, k = 16, fp32 9.0 -> 8.6; 64 x 4096 -> 11008, k = 256, bf16 29.2 -> 17.9; 128 x 8192 -> 1024, k = 128, bf16 28.0 -> 15.2;
+// 1 x 4096 -> 4096, k = 16, fp32: even (8.6 to 9.0 either way); 64 x 4096 -> 11008, k = 256, bf16 29.2 -> 17.9; 128 x 8192 -> 1024, k = 128, bf16 28.0 -> 15.2;
 // 256 x 512 -> 512, k = 128, fp32 17.4 -> 9.8.  What is left is launches and memory round trips: x in, partial sums out and in, y out.
 // Tokens split finer than they were (48 to a block of either kind): 48 x 768 -> 3072, k = 256, bf16 15.5 -> 10.7, 32 tokens 13.6 -> 10.6.
 //
@@ -537,7 +537,8 @@ static FewPlan few_plan(const rdb_linear_desc *d)
 // 128 x 512 -> 4096, k = 256 (512 units): 12.8 -> 13.1; 64 tokens (256): 12.4 -> 10.1.
 // Beyond 256 tokens only contractions of 512 and more, where the other kernels' one block a tile takes longest: 512 x 2048 -> 2048, k = 64: 19.0 ->
 // 13.2, fp32 18.5 -> 15.1; 512 x 8192 -> 512, k = 16: 30.9 -> 11.5 and 21.1 -> 13.0; 512 x 4096 -> 512, k = 128: 28.7 -> 18.9, fp32 24.0 -> 24.6; 512 x
-// 520 -> 2000, k = 64: 12.0 -> 11.2; 640 tokens x 1001 -> 999, k = 60: 16.2 -> 17.4.  For shorter ones y stays bit for bit that of the forms that keep z.
+// 520 -> 2000, k = 64: 12.0 -> 11.2; 640 tokens x 1001 -> 999, k = 60: 16.2 -> 17.4.  In bf16 y is not bit for bit that of the forms that keep z
+// for a backward pass (rounded to bf16, and multiplied as it is kept): z stays in fp32 here, and y is nearer to 64 bits.
 // The factored form is taken as far as everywhere: up to 16 times the products of one with a stored weight.
 static bool few_pays(const rdb_linear_desc *d)
 {

@@ -581,7 +581,7 @@ extern "C" int rdb_linear_fwd(void *y, int64_t ldy, const void *x, int64_t ldx, 
     }
     if (d->algo == RDB_ALGO_AUTO && d->act_dtype == RDB_BF16) {
         // bf16 requests that kept every kernel above away (rows that are not 16-byte aligned, ...): the same kernels, reading bf16
-        // value by value
+        // at any address
         rc = linear_fwd_f32(y, ldy, x, ldx, coef, scale_bias, bias, d, num_compute_units(), workspace, workspace_bytes, s);
         if (rc != RDB_E_UNSUPPORTED) return rc;
     }

@@ -111,6 +111,25 @@ def test_fp32_products_where_they_are_asked_for(T, in_f, out_f, k):
     assert torch.equal(call(_lib.RDB_ALGO_AUTO), split)
 
 
+@pytest.mark.parametrize("T,in_f,out_f,k", [(97, 2048, 512, 64), (128, 4096, 1024, 256), (300, 1024, 2048, 128), (500, 8192, 512, 16), (16, 1024, 1024, 384)])
+def test_evaluation_and_training_in_bf16(T, in_f, out_f, k):
+    """A forward that keeps z for a backward pass keeps it in bf16 and multiplies what it keeps; one that keeps nothing goes on with z in
+    fp32.  So y differs: by z's rounding and its own, each 2^-9 of a value at most either way (1.7e-3 of a result in the 2-norm), and
+    evaluation is the nearer one to 64 bits."""
+    from randumb_amd import SillyLinear
+
+    x, c, _, N = _case(T, in_f, out_f, k, torch.bfloat16)
+    layer = SillyLinear(in_f, out_f, [k, k], [5, 6], bias=False, device="cuda", dtype=torch.bfloat16, matrix_coef=True)
+    with torch.no_grad():
+        layer.weight_coef.copy_(c)
+        evaluated = layer(x)
+    trained = layer(x.requires_grad_())
+    assert "Projected" in repr(trained.grad_fn)
+    want = (x.detach().double() @ N) @ c.double().t()
+    e, t = _rel(evaluated, want), _rel(trained.detach(), want)
+    assert e < t < 4e-3 and e < 2e-3 and _rel(evaluated, trained.detach().double()) < 4e-3
+
+
 def test_recorded_launches():
     """Both forms recorded into one graph and replayed on changing inputs, with eager calls in between."""
     shapes = [(5, 1001, 999, 99), (100, 264, 352, 64), (16, 4096, 4096, 256), (40, 8192, 512, 512)]   # one launch (one group of tokens, four), two, three

@@ -53,7 +53,7 @@ __global__ __launch_bounds__(NT) void sq5_fill_1d_kernel(float *__restrict__ out
 constexpr int COEF_CHUNK = 2048;
 // Coefficients below this in magnitude: 2^31 times their terms stays finite, and so do sums of them; others (and NaNs) get the factor 2^-31
 // term by term.  Without it, and with MAT_UNROLL terms a turn of the loop (still one after the other), a term takes 17 vector instructions
-// instead of 19: 768 x 3072 elements, k = 256: 219 -> 205 us, and the pass of that layer, 1024 tokens, 538 -> 520; 4096 rows of a 50304 x
+// instead of 19: 768 x 3072 elements, k = 256: 219 -> 205 us, and the pass of that layer, 1024 tokens, 538 -> 520 (another box: 558 -> 550); 4096 rows of a 50304 x
 // 768 table, forward and backward, 525 -> 522 (one term a turn: 540).  The round constants stay literals: in scalar or vector registers the
 // same instructions take 2 to 6 % longer.  What is left of a chunk goes by fours and twos.  The look at the coefficients costs a launch about
 // a microsecond, which up to MAT_SHORT terms are not paid back: those get the factor term by term.  768 x 3072 elements, term by term

@@ -328,7 +328,7 @@ Tensor once_differentiable(const char *who, const Tensor &grad, const Tensor &dy
     for (int i : inputs)
         if (node && i >= 0 && i < (int)node->num_outputs()) depends_on(node->next_edge(i));
     if (edges.empty()) return grad;   // a constant
-    const Tensor out = grad.detach();
+    const Tensor out = grad.tensor_data();
     torch::autograd::set_history(out, std::make_shared<torch::autograd::Error>(std::string(who) + " has no second derivative", std::move(edges)));
     return out;
 }

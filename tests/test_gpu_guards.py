@@ -275,6 +275,12 @@ def test_second_derivatives_of_a_matrix_layer_raise(form, python, monkeypatch):
     (g,) = torch.autograd.grad((layer(s.square()).float() ** 2).sum(), s, create_graph=True)
     with pytest.raises(RuntimeError, match="second derivative"):
         torch.autograd.grad(g.float().sum(), s)
+    # the gradients that a program accumulates under create_graph can be cleared in place
+    for gradient in (dy, w):
+        layer(x).backward(gradient, create_graph=True)
+        layer.zero_grad(set_to_none=False)
+        assert not bool(layer.weight_coef.grad.any()) and layer.weight_coef.grad.grad_fn is None
+    layer.zero_grad(set_to_none=True)
     # nothing to come: constants, as they were
     layer.requires_grad_(False)
     (g,) = torch.autograd.grad(layer(x), x, dy, create_graph=True)

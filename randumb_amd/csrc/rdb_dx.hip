@@ -281,10 +281,10 @@ __global__ __launch_bounds__(256, 2) void bwd_tn_red_kernel(BwdBParams p)
 }
 
 // dx = t . N for k <= 256 with t held in registers (rdb_stationary.hpp), alone and beside the reduction blocks.
-template <int KG> __global__ __launch_bounds__(ST_THREADS, 1) void dx_tns_kernel(StParams p)
+template <int KG, int AUX> __global__ __launch_bounds__(ST_THREADS, 1) void dx_tns_kernel(StParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    stationary_block<KG, false, true, true>(p, smem_raw, blockIdx.x);
+    stationary_block<KG, false, true, AUX, true>(p, smem_raw, blockIdx.x);
 }
 
 struct BwdBsParams {
@@ -293,11 +293,11 @@ struct BwdBsParams {
     int tn_blocks;
 };
 
-template <int KG> __global__ __launch_bounds__(ST_THREADS, 1) void bwd_tns_red_kernel(BwdBsParams p)
+template <int KG, int AUX> __global__ __launch_bounds__(ST_THREADS, 1) void bwd_tns_red_kernel(BwdBsParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     if ((int)blockIdx.x < p.tn_blocks)
-        stationary_block<KG, false, true, true>(p.tn, smem_raw, blockIdx.x);
+        stationary_block<KG, false, true, AUX, true>(p.tn, smem_raw, blockIdx.x);
     else
         red_block(p.red, blockIdx.x - p.tn_blocks, gridDim.x - p.tn_blocks);
 }
@@ -419,13 +419,9 @@ int linear_dx_factored(void *dx, int64_t lddx, const void *dy, int64_t lddy, con
     if (stationary) {
         StParams q;
         const int items = make_tns_params(q, dx, lddx, workspace, d, num_cus);
-        const size_t smem = stationary_smem(kg);
-        switch (kg) {
-        case 1: return launch_stationary(dx_tns_kernel<1>, q, items, smem, s, "dx_tns_kernel<1>");
-        case 2: return launch_stationary(dx_tns_kernel<2>, q, items, smem, s, "dx_tns_kernel<2>");
-        case 3: return launch_stationary(dx_tns_kernel<3>, q, items, smem, s, "dx_tns_kernel<3>");
-        default: return launch_stationary(dx_tns_kernel<4>, q, items, smem, s, "dx_tns_kernel<4>");
-        }
+        return with_stationary_variant(q, [&](auto kgc, auto aux) {
+            return launch_stationary(dx_tns_kernel<decltype(kgc)::value, decltype(aux)::value>, q, items, stationary_smem(kgc), s, "dx_tns_kernel");
+        });
     }
     TNParams p2;
     const int items = make_tn_params(p2, dx, lddx, workspace, d);
@@ -519,19 +515,13 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             if (bs.tn_blocks < num_cus && rblocks > num_cus - bs.tn_blocks) rblocks = num_cus - bs.tn_blocks;
             if (rblocks < 1) rblocks = 1;
             if (direct) rblocks = 0;
-            const int kg = (int)cdiv(d->k, 64);
-            const size_t smem_s = stationary_smem(kg);
-            const void *fn = kg == 1 ? (const void *)bwd_tns_red_kernel<1> : kg == 2 ? (const void *)bwd_tns_red_kernel<2>
-                           : kg == 3 ? (const void *)bwd_tns_red_kernel<3> : (const void *)bwd_tns_red_kernel<4>;
-            if (int rl = reserve_lds(fn, smem_s, "bwd_tns_red_kernel")) return rl;
-            const dim3 grid(bs.tn_blocks + rblocks), block(ST_THREADS);
-            switch (kg) {
-            case 1: bwd_tns_red_kernel<1><<<grid, block, smem_s, s>>>(bs); break;
-            case 2: bwd_tns_red_kernel<2><<<grid, block, smem_s, s>>>(bs); break;
-            case 3: bwd_tns_red_kernel<3><<<grid, block, smem_s, s>>>(bs); break;
-            default: bwd_tns_red_kernel<4><<<grid, block, smem_s, s>>>(bs); break;
-            }
-            return check_launch("bwd_tns_red_kernel");
+            return with_stationary_variant(bs.tn, [&](auto kg, auto aux) {
+                auto kernel = bwd_tns_red_kernel<decltype(kg)::value, decltype(aux)::value>;
+                const size_t smem_s = stationary_smem(kg);
+                if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem_s, "bwd_tns_red_kernel")) return rl;
+                kernel<<<bs.tn_blocks + rblocks, ST_THREADS, smem_s, s>>>(bs);
+                return check_launch("bwd_tns_red_kernel");
+            });
         }
         const int64_t table = dx_big_table_bytes(d, num_cus);
         if (direct && table && workspace_bytes >= base + table) {   // nothing to add up, and room for N^T

@@ -379,10 +379,10 @@ __global__ __launch_bounds__(256, 2) void factored_y_kernel(YParams p)
 // ----------------------------------------------------------------------------------------------- y = z . C^T, k <= 256
 // body in rdb_stationary.hpp: the projection of a token stays in registers (read in fragment order, as factored_z_kernel
 // leaves it), the rows of C stream through LDS
-template <int KG, bool BIAS> __global__ __launch_bounds__(ST_THREADS, 1) void factored_ys_kernel(StParams p)
+template <int KG, bool BIAS, int AUX> __global__ __launch_bounds__(ST_THREADS, 1) void factored_ys_kernel(StParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    stationary_block<KG, BIAS, false, true>(p, smem_raw, blockIdx.x);
+    stationary_block<KG, BIAS, false, AUX, true>(p, smem_raw, blockIdx.x);
 }
 
 // Projection and forward product in one launch: blocks 0 .. z_grid - 1 project (z_block), the next c_blocks transpose C, the others multiply
@@ -394,7 +394,7 @@ struct ZYParams {
     StParams y;
 };
 
-template <int KG, bool BIAS> __global__ __launch_bounds__(ST_THREADS, 1) void factored_zy_kernel(ZYParams p)
+template <int KG, bool BIAS, int AUX> __global__ __launch_bounds__(ST_THREADS, 1) void factored_zy_kernel(ZYParams p)
 {
     static_assert(KZ_THREADS == ST_THREADS && KZ_BT == ST_BT, "one block size and one token tile for both kinds of block");
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -404,7 +404,7 @@ template <int KG, bool BIAS> __global__ __launch_bounds__(ST_THREADS, 1) void fa
     else if (block < p.z.c_blocks)
         transpose_units(p.z, block * (KZ_THREADS / 64) + (int)(threadIdx.x >> 6), p.z.c_blocks * (KZ_THREADS / 64));
     else
-        stationary_block<KG, BIAS, false, true>(p.y, smem_raw, block - p.z.c_blocks);
+        stationary_block<KG, BIAS, false, AUX, true>(p.y, smem_raw, block - p.z.c_blocks);
 }
 
 // ----------------------------------------------------------------------------------------------- dC = dy^T . z
@@ -572,12 +572,22 @@ static int fill_ys_params(StParams &q, void *y, int64_t ldy, const void *state, 
     return make_stationary_grid(q, d->tokens, d->out_f, num_cus);
 }
 
-template <int KG, bool BIAS> static int launch_zy(const ZYParams &p, int y_items, hipStream_t s)
+template <bool BIAS> static int launch_zy(const ZYParams &p, int y_items, hipStream_t s)
 {
-    const size_t smem = std::max(z_smem(), stationary_smem(KG));
-    if (int rl = reserve_lds(reinterpret_cast<const void *>(factored_zy_kernel<KG, BIAS>), smem, "factored_zy_kernel")) return rl;
-    factored_zy_kernel<KG, BIAS><<<p.z.z_grid + p.z.c_blocks + xcd_grid_size(y_items), ST_THREADS, smem, s>>>(p);
-    return check_launch("factored_zy_kernel");
+    return with_stationary_variant(p.y, [&](auto kg, auto aux) {
+        auto kernel = factored_zy_kernel<decltype(kg)::value, BIAS, decltype(aux)::value>;
+        const size_t smem = std::max(z_smem(), stationary_smem(kg));
+        if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem, "factored_zy_kernel")) return rl;
+        kernel<<<p.z.z_grid + p.z.c_blocks + xcd_grid_size(y_items), ST_THREADS, smem, s>>>(p);
+        return check_launch("factored_zy_kernel");
+    });
+}
+
+template <bool BIAS> static int launch_ys(const StParams &q, int items, hipStream_t s)
+{
+    return with_stationary_variant(q, [&](auto kg, auto aux) {
+        return launch_stationary(factored_ys_kernel<decltype(kg)::value, BIAS, decltype(aux)::value>, q, items, stationary_smem(kg), s, "factored_ys_kernel");
+    });
 }
 
 // state <- projection of x (with the transposed coefficients if with_ct), y <- forward product, in one launch when the
@@ -609,21 +619,7 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
     const bool spread = spread_ranges(p.z, state, y, ldy, d, &rc);
     if (rc) return rc;
     set_z_grid(p.z, xcd_grid_size(p.z.tiles_m * p.z.tiles_t) * (spread ? p.z.ranges : 1), num_cus);
-    const int kg = (int)cdiv(d->k, 64);
-    if (bias) {
-        switch (kg) {
-        case 1: return launch_zy<1, true>(p, y_items, s);
-        case 2: return launch_zy<2, true>(p, y_items, s);
-        case 3: return launch_zy<3, true>(p, y_items, s);
-        default: return launch_zy<4, true>(p, y_items, s);
-        }
-    }
-    switch (kg) {
-    case 1: return launch_zy<1, false>(p, y_items, s);
-    case 2: return launch_zy<2, false>(p, y_items, s);
-    case 3: return launch_zy<3, false>(p, y_items, s);
-    default: return launch_zy<4, false>(p, y_items, s);
-    }
+    return bias ? launch_zy<true>(p, y_items, s) : launch_zy<false>(p, y_items, s);
 }
 
 // Test hook: only the multiplying blocks of the one-launch forward, waiting (at most `polls` polls each) for a tag that
@@ -640,14 +636,7 @@ int selftest_giveup_factored(void *y, int64_t ldy, void *state, const void *coef
     q.sync_wait.err = reinterpret_cast<unsigned int *>(state) + 1;
     q.sync_wait.polls = polls;
     if (int rc = sync_giveups_ptr(&q.sync_wait.giveups)) return rc;
-    const int kg = (int)cdiv(d->k, 64);
-    const size_t smem = stationary_smem(kg);
-    switch (kg) {
-    case 1: return launch_stationary(factored_ys_kernel<1, false>, q, items, smem, s, "factored_ys_kernel<1> (self-test)");
-    case 2: return launch_stationary(factored_ys_kernel<2, false>, q, items, smem, s, "factored_ys_kernel<2> (self-test)");
-    case 3: return launch_stationary(factored_ys_kernel<3, false>, q, items, smem, s, "factored_ys_kernel<3> (self-test)");
-    default: return launch_stationary(factored_ys_kernel<4, false>, q, items, smem, s, "factored_ys_kernel<4> (self-test)");
-    }
+    return launch_ys<false>(q, items, s);
 }
 
 int linear_fwd_projected(void *y, int64_t ldy, const void *state, const void *coef, const void *bias, const rdb_linear_desc *d, int num_cus,
@@ -660,22 +649,7 @@ int linear_fwd_projected(void *y, int64_t ldy, const void *state, const void *co
         StParams q;
         const int items = fill_ys_params(q, y, ldy, state, coef, bias, d, num_cus);
         if (!items) return RDB_E_UNSUPPORTED;
-        const int kg = (int)cdiv(d->k, 64);
-        const size_t smem = stationary_smem(kg);
-        if (bias) {
-            switch (kg) {
-            case 1: return launch_stationary(factored_ys_kernel<1, true>, q, items, smem, s, "factored_ys_kernel<1,bias>");
-            case 2: return launch_stationary(factored_ys_kernel<2, true>, q, items, smem, s, "factored_ys_kernel<2,bias>");
-            case 3: return launch_stationary(factored_ys_kernel<3, true>, q, items, smem, s, "factored_ys_kernel<3,bias>");
-            default: return launch_stationary(factored_ys_kernel<4, true>, q, items, smem, s, "factored_ys_kernel<4,bias>");
-            }
-        }
-        switch (kg) {
-        case 1: return launch_stationary(factored_ys_kernel<1, false>, q, items, smem, s, "factored_ys_kernel<1>");
-        case 2: return launch_stationary(factored_ys_kernel<2, false>, q, items, smem, s, "factored_ys_kernel<2>");
-        case 3: return launch_stationary(factored_ys_kernel<3, false>, q, items, smem, s, "factored_ys_kernel<3>");
-        default: return launch_stationary(factored_ys_kernel<4, false>, q, items, smem, s, "factored_ys_kernel<4>");
-        }
+        return bias ? launch_ys<true>(q, items, s) : launch_ys<false>(q, items, s);
     }
     if (big_fwd_applies(d, num_cus)) return linear_fwd_big(y, ldy, state, coef, bias, d, num_cus, s);
     YParams p;

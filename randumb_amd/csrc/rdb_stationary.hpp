@@ -12,13 +12,16 @@
 #pragma once
 #include "rdb_gemm.hpp"
 #include "rdb_tile.hpp"
+#include <type_traits>
 
 namespace rdb {
 
-#ifndef RDB_Y_STORE_AUX
-#define RDB_Y_STORE_AUX 2   // cache policy of the output row stores: non-temporal (y and dx are not read again by this library, and
-                           // lines that do not linger in L2 need no write-back when the kernel ends: the next launch starts sooner)
-#endif
+// Cache policy of the output row stores where rows are whole lines of 128 bytes: non-temporal (y and dx are not read again by this library,
+// and lines that do not linger in L2 need no write-back when the kernel ends: the next launch starts sooner; 8192 tokens x 768 -> 3072,
+// forward 27.0 us, with plain stores 29.4).  Other rows leave with plain stores: a pair of neighbouring 128-byte pieces shares a line there, and a
+// streamed part of a line is a read and a write of memory (7186 tokens x 264 -> 5384: forward 63.5 -> 30.6 us; 4096 x 264 -> 5400: 33.6 -> 18;
+// -> 5408, halves of lines: 18.4 -> 17.4; -> 5440, whole lines: 17.0 streamed, 17.2 plain; dx of 4096 x 3208 -> 520: 16.4 -> 8.9).
+constexpr int Y_STREAM = 2;
 
 constexpr int ST_BT = 256, ST_BO = 64, ST_STG_LD = ST_BO + 8, ST_WAVES = 8, ST_THREADS = ST_WAVES * 64, ST_TW = ST_BT / ST_WAVES;
 constexpr int ST_KMAX = 256;
@@ -43,8 +46,9 @@ struct StParams {
 
 // KG: k rounded up to groups of 64 (compile time: the k loop is one straight line of code).  NOISE: the right operand's
 // rows are 2^31 * noise(PRIME*row + m), hashed into the tile; the producer of the left operand has scaled it by 2^-31
-// (exact in bf16).
-template <int KG, bool BIAS, bool NOISE> struct StBlock {
+// (exact in bf16).  AUX: cache policy of the row stores (an immediate of the instruction: two copies of the steps in one kernel cost it 10 to 20
+// registers, and spills with k = 256 and a bias).
+template <int KG, bool BIAS, bool NOISE, int AUX> struct StBlock {
     static constexpr int kpad = KG * 64, ldk = kpad + 8, cpr = kpad / 8, ncp = ST_BO * cpr, NQ = ncp / ST_THREADS;
     const StParams &p;
     bf16_t *Cs;   // [2][64 rows][ldk]
@@ -146,7 +150,7 @@ template <int KG, bool BIAS, bool NOISE> struct StBlock {
                     const int qq = h * 2 + q;
                     const uint32_t a = (o0 + (lane & 7) * 8 < p.out_f && tok_y + qq * 8 < p.tokens)
                                            ? off_y + (uint32_t)(qq * 8 * (int)p.ldy * 2 + o0 * 2) : BUFFER_OOB;
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v[q]), rs_y, (int)a, 0, RDB_Y_STORE_AUX);
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v[q]), rs_y, (int)a, 0, AUX);
                 }
                 if (op == 9) __builtin_amdgcn_wave_barrier();
             }
@@ -197,10 +201,10 @@ template <int KG, bool BIAS, bool NOISE> struct StBlock {
 };
 
 // `block`: index of this block among the blocks that run this body; all ST_THREADS threads of the block must call.
-template <int KG, bool BIAS, bool NOISE, bool ZFRAG = false>
+template <int KG, bool BIAS, bool NOISE, int AUX, bool ZFRAG = false>
 __device__ __forceinline__ void stationary_block(const StParams &p, unsigned char *smem_raw, int block)
 {
-    typedef StBlock<KG, BIAS, NOISE> B;
+    typedef StBlock<KG, BIAS, NOISE, AUX> B;
     const int t = threadIdx.x, wave = t >> 6;
     // work item = (token tile, split), split fastest: neighbours share the left operand's tile, everyone shares the right operand
     const int w = xcd_work_item(block, p.tiles_t * p.splits);
@@ -351,6 +355,21 @@ inline int make_stationary_grid(StParams &q, int64_t tokens, int64_t out_f, int 
     q.units_per_split = (int)cdiv(units, splits);
     q.splits = (int)cdiv(units, q.units_per_split);
     return q.tiles_t * q.splits;
+}
+
+// f(k in groups of 64, cache policy of the row stores), both as std::integral_constant, for [tokens x out_f] with k coefficients
+template <class F> inline int with_stationary_variant(const StParams &q, F &&f)
+{
+    auto with_kg = [&](auto aux) {
+        switch (cdiv(q.k, 64)) {
+        case 1: return f(std::integral_constant<int, 1>{}, aux);
+        case 2: return f(std::integral_constant<int, 2>{}, aux);
+        case 3: return f(std::integral_constant<int, 3>{}, aux);
+        default: return f(std::integral_constant<int, 4>{}, aux);
+        }
+    };
+    const bool whole_lines = q.ldy % 64 == 0 && ((uintptr_t)q.y & 127) == 0;
+    return whole_lines ? with_kg(std::integral_constant<int, Y_STREAM>{}) : with_kg(std::integral_constant<int, 0>{});
 }
 
 template <class K> inline int launch_stationary(K kernel, const StParams &q, int items, size_t smem, hipStream_t s, const char *name)

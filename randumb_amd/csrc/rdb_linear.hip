@@ -356,10 +356,11 @@ int64_t linear_bwd_projected_extra(const rdb_linear_desc *d, int num_cus);
 int linear_dx_rbias_add(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table = nullptr, int64_t table_bytes = 0);
 int linear_fwd_rbias_add(void *y, int64_t ldy, const void *x, int64_t ldx, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table = nullptr, int64_t table_bytes = 0);
 int64_t linear_dx_rbias_dot_floats(const rdb_linear_desc *d);
-int linear_dx_rbias_add_dscale(void *dx, int64_t lddx, float *dscale, float *dot_part, const void *dy, int64_t lddy, const void *x, int64_t ldx,
-                               const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table = nullptr, int64_t table_bytes = 0);
+int linear_dx_rbias_add_dscale(void *dx, int64_t lddx, void *dscale, int dscale_dtype, float *dot_part, const void *dy, int64_t lddy, const void *x,
+                               int64_t ldx, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table = nullptr, int64_t table_bytes = 0);
 // rdb_big.hip
 int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);
+int64_t rbias_scratch_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);   // rdb_rbias.hip
 int linear_project_before(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, int num_cus,
                           hipStream_t s);   // rdb_factored.hip
 int linear_fwd_rbias_big(void *y, int64_t ldy, const void *x, int64_t ldx, const void *state, const void *coef, const void *scale, const void *bias,
@@ -484,12 +485,12 @@ static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d)
     }
     if (op == RDB_OP_LINEAR_RBIAS_BWD || op == RDB_OP_LINEAR_RBIAS_BWD_FULL) {   // one float per tile of the random-bias product (the gradient of the scale)
         if (d->act_dtype != RDB_BF16 || d->coef_dtype != RDB_BF16 || d->in_f % 8 || d->out_f % 8) return 0;
-        const int64_t table = op == RDB_OP_LINEAR_RBIAS_BWD_FULL ? rbias_big_table_bytes(d, d->in_f, num_compute_units()) : 0;
-        return table > 0 ? rbias_dot_room(d) + table : linear_dx_rbias_dot_floats(d) * 4;   // ... and R behind them
+        const int64_t more = op == RDB_OP_LINEAR_RBIAS_BWD_FULL ? rbias_scratch_bytes(d, d->in_f, num_compute_units()) : 0;
+        return more > 0 ? rbias_dot_room(d) + more : linear_dx_rbias_dot_floats(d) * 4;   // ... and behind them R, or sums of ranges
     }
     if (op == RDB_OP_LINEAR_PROJECT_FWD_RBIAS) return project_fwd_rbias_table(d);
     if (op == RDB_OP_LINEAR_RBIAS_FWD)
-        return d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16 ? rbias_big_table_bytes(d, d->out_f, num_compute_units()) : 0;
+        return d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16 ? rbias_scratch_bytes(d, d->out_f, num_compute_units()) : 0;
     if (op == RDB_OP_LINEAR_BWD_PROJECTED || op == RDB_OP_LINEAR_BWD_PROJECTED_TO) {
         const int64_t base = bwd_projected_workspace(d, op == RDB_OP_LINEAR_BWD_PROJECTED_TO), extra = base > 0 ? bwd_projected_extra(d) : 0;
         return extra > 0 ? (base + 255) / 256 * 256 + extra : base;   // what lies behind `base` is never required
@@ -710,7 +711,7 @@ extern "C" int rdb_linear_bwd_dx_dscale(void *dx, int64_t lddx, float *d_scale_b
     if (rc == RDB_E_UNSUPPORTED) return set_error(RDB_E_UNSUPPORTED, "%s", why);
     if (rc) return rc;
     float *dots = reinterpret_cast<float *>(static_cast<char *>(workspace) + t_bytes);
-    rc = linear_dx_rbias_add_dscale(dx, lddx, d_scale_bias, dots, dy, lddy, x, ldx, scale_bias, d, s);
+    rc = linear_dx_rbias_add_dscale(dx, lddx, d_scale_bias, RDB_F32, dots, dy, lddy, x, ldx, scale_bias, d, s);
     if (rc == RDB_E_UNSUPPORTED) return set_error(RDB_E_UNSUPPORTED, "%s", why);
     return rc;
 }
@@ -765,7 +766,7 @@ extern "C" int rdb_linear_rbias_bwd(void *dx, int64_t lddx, float *d_scale_bias,
     const int64_t need = linear_dx_rbias_dot_floats(d) * 4;
     if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 3))
         return set_error(RDB_E_WORKSPACE, "rdb_linear_rbias_bwd: the gradient of the scale needs a workspace of %lld bytes", (long long)need);
-    rc = linear_dx_rbias_add_dscale(dx, lddx, d_scale_bias, static_cast<float *>(workspace), dy, lddy, x, ldx, scale_bias, d, s, table, room);
+    rc = linear_dx_rbias_add_dscale(dx, lddx, d_scale_bias, RDB_F32, static_cast<float *>(workspace), dy, lddy, x, ldx, scale_bias, d, s, table, room);
     return rc == RDB_E_UNSUPPORTED ? set_error(RDB_E_UNSUPPORTED, "%s", why) : rc;
 }
 

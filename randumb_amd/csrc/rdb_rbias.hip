@@ -67,16 +67,27 @@ struct RBiasParams {
     const bf16_t *other;
     int64_t ld_other;
     float *dot_part;
+    // RB_PART: the contraction in `ranges` ranges of range_stages stages, a block per tile and range.  Sums (without s): for each range and
+    // tile the accumulators as the lanes hold them, [wave][feature block][token block][quad][lane][4]
+    int ranges, range_stages;
+    float *part;
 };
+enum { RB_ADD = 0, RB_ADD_DOT = 1, RB_PART = 2 };
+constexpr int RB_TILE = RB_BI * RB_BT;
 
-template <bool DOT> __global__ __launch_bounds__(256, 2) void rbias_add_kernel(RBiasParams p)
+template <int MODE> __global__ __launch_bounds__(256, 2) void rbias_add_kernel(RBiasParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
-    // work item = (token tile, feature tile), feature tile fastest: neighbours share the dy tile
-    const int w = xcd_work_item(blockIdx.x, p.tiles_i * p.tiles_t);
-    if (w >= p.tiles_i * p.tiles_t) return;
+    constexpr bool DOT = MODE == RB_ADD_DOT;
+    // work item = (range, token tile, feature tile), feature tile fastest: neighbours share the dy tile
+    const int tiles = p.tiles_i * p.tiles_t, items = MODE == RB_PART ? tiles * p.ranges : tiles;
+    const int item = xcd_work_item(blockIdx.x, items);
+    if (item >= items) return;
+    const int range = MODE == RB_PART ? item / tiles : 0, w = item - range * tiles;
     const int i0 = (w % p.tiles_i) * RB_BI, tok0 = (w / p.tiles_i) * RB_BT;
+    const int s_begin = MODE == RB_PART ? range * p.range_stages : 0, all = (p.out_f + RB_BK - 1) / RB_BK;
+    const int s_end = MODE == RB_PART ? min(all, s_begin + p.range_stages) : all;
     constexpr int MI = RB_BI / 32, NI = RB_BT / 128;
     f32x16 acc[MI][NI];
 #pragma unroll
@@ -85,9 +96,22 @@ template <bool DOT> __global__ __launch_bounds__(256, 2) void rbias_add_kernel(R
         for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = zero16();
     // "A": 2^31 * R, rows = columns of dst: the noise index moves by sR per row and by sK per contraction value
     Noise1DOperand<RB_BI, RB_BK> opr = {i0, p.sR, p.sK, p.seed};
-    // "B": src[tok][c]; contraction values past the end read as zeros, whatever the hash says there
-    GlobalOperand<RB_BT, RB_BK, K_CONT> opdy = {p.dy, p.lddy, tok0, p.tokens, p.out_f, (int64_t)(p.tokens - 1) * p.lddy + p.out_f};
-    gemm_mainloop<RB_BI, RB_BT, RB_BK, 1, 2, 1>(acc, lds, opr, opdy, 0, (p.out_f + RB_BK - 1) / RB_BK);
+    // "B": src[tok][c]; contraction values past the end (of the range) read as zeros, whatever the hash says there
+    GlobalOperand<RB_BT, RB_BK, K_CONT> opdy = {p.dy, p.lddy, tok0, p.tokens, min(p.out_f, s_end * RB_BK), (int64_t)(p.tokens - 1) * p.lddy + p.out_f};
+    gemm_mainloop<RB_BI, RB_BT, RB_BK, 1, 2, 1>(acc, lds, opr, opdy, s_begin * RB_BK, s_end - s_begin);
+    if constexpr (MODE == RB_PART) {
+        constexpr float unit = 4.656612873077392578125e-10f;
+        f32x4 *dst = reinterpret_cast<f32x4 *>(p.part + (int64_t)item * RB_TILE) + threadIdx.x / 64 * (MI * NI * 4 * 64) + threadIdx.x % 64;
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+                for (int jq = 0; jq < 4; ++jq)
+                    dst[((mi * NI + ni) * 4 + jq) * 64] = f32x4{acc[mi][ni][jq * 4] * unit, acc[mi][ni][jq * 4 + 1] * unit, acc[mi][ni][jq * 4 + 2] * unit,
+                                                                acc[mi][ni][jq * 4 + 3] * unit};
+        return;
+    }
     // dx += s * (2^-31 * acc), through LDS as fp32 so that every lane updates 8 consecutive features of a token's row
     // (2^-31 * acc is exact, so the product with s is rounded once, as s * 2^-31 times acc would be)
     const float sval = bf16_to_f32(*p.scale_bias);
@@ -156,6 +180,61 @@ template <bool DOT> __global__ __launch_bounds__(256, 2) void rbias_add_kernel(R
         if (lane == 0) wsum[wave] = dot;
         __syncthreads();
         if (t == 0) p.dot_part[w] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+    }
+}
+
+// dst += s * (the ranges' sums, added up in range order); DOT: and their product with `other`, one sum per block.  A block takes 32 tokens
+// of a tile, a thread 8 features of a token: two quads of the lanes that hold them, and whole rows of 128 bytes in dst.
+template <bool DOT> __global__ __launch_bounds__(256) void rbias_sum_ranges_kernel(RBiasParams p)
+{
+    constexpr int NI = RB_BT / 128, SUBS = RB_BT / 32;
+    const int t = threadIdx.x, w = blockIdx.x / SUBS, sub = blockIdx.x % SUBS, wave = sub / NI, ni = sub % NI;
+    const int r = t >> 3, c = t & 7, tok = w / p.tiles_i * RB_BT + sub * 32 + r, a = w % p.tiles_i * RB_BI + c * 8;
+    const bool live = tok < p.tokens && a < p.in_f;   // in_f is a multiple of 8: a piece lies inside or outside
+    const int64_t at = (int64_t)tok * p.lddx + a;
+    float dot = 0.0f;
+    if (live) {
+        Frag8 old, ot;
+        old.f4 = *reinterpret_cast<const f32x4 *>(p.dx + at);
+        if (DOT) ot.f4 = *reinterpret_cast<const f32x4 *>(p.other + (int64_t)tok * p.ld_other + a);
+        const float sval = bf16_to_f32(*p.scale_bias);
+        const f32x4 *src = reinterpret_cast<const f32x4 *>(p.part + (int64_t)w * RB_TILE) + ((wave * (RB_BI / 32) + (c >> 2)) * NI + ni) * 4 * 64 + (c & 3) * 64 + r;
+        const int64_t stride = (int64_t)p.tiles_i * p.tiles_t * (RB_TILE / 4);
+        f32x4 lo = src[0], hi = src[32];
+        for (int r0 = 1; r0 < p.ranges; r0 += 4) {   // four ranges' loads in flight
+            f32x4 l[4], h[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t o = min(r0 + j, p.ranges - 1) * stride;   // clamped: loaded, not added
+                l[j] = src[o];
+                h[j] = src[o + 32];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (r0 + j < p.ranges) {
+                    lo += l[j];
+                    hi += h[j];
+                }
+        }
+        Frag8 nw;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float v0 = e < 2 ? lo[2 * e] : hi[2 * e - 4], v1 = e < 2 ? lo[2 * e + 1] : hi[2 * e - 3];
+            if (DOT) {
+                dot = fmaf(v0, __uint_as_float(ot.u[e] << 16), dot);
+                dot = fmaf(v1, __uint_as_float(ot.u[e] & 0xffff0000u), dot);
+            }
+            nw.u[e] = f32x2_to_bf16x2(__uint_as_float(old.u[e] << 16) + sval * v0, __uint_as_float(old.u[e] & 0xffff0000u) + sval * v1);
+        }
+        *reinterpret_cast<f32x4 *>(p.dx + at) = nw.f4;
+    }
+    if (DOT) {   // lanes, then waves, in a fixed order
+        __shared__ float wsum[4];
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) dot += __shfl_xor(dot, off, 64);
+        if ((t & 63) == 0) wsum[t >> 6] = dot;
+        __syncthreads();
+        if (t == 0) p.dot_part[blockIdx.x] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
     }
 }
 
@@ -359,7 +438,7 @@ template <bool DOT> __global__ __launch_bounds__(RW_THREADS, 1) void rbias_wide_
 }
 
 // out[0] = part[0] + ... + part[n - 1], in a fixed order (one block)
-__global__ __launch_bounds__(256) void rbias_sum_kernel(float *__restrict__ out, const float *__restrict__ part, int n)
+template <typename T> __global__ __launch_bounds__(256) void rbias_sum_kernel(T *__restrict__ out, const float *__restrict__ part, int n)
 {
     __shared__ float sh[256];
     float v = 0.0f;
@@ -370,17 +449,66 @@ __global__ __launch_bounds__(256) void rbias_sum_kernel(float *__restrict__ out,
         if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[0] = sh[0];
+    if (threadIdx.x == 0) {
+        if constexpr (sizeof(T) == 2) out[0] = f32_to_bf16(sh[0]);
+        else out[0] = sh[0];
+    }
+}
+static int launch_rbias_sum(void *out, int dtype, const float *part, int n, hipStream_t s)
+{
+    if (dtype == RDB_BF16) rbias_sum_kernel<bf16_t><<<1, 256, 0, s>>>(static_cast<bf16_t *>(out), part, n);
+    else rbias_sum_kernel<float><<<1, 256, 0, s>>>(static_cast<float *>(out), part, n);
+    return check_launch("rbias_sum_kernel");
 }
 
 // floats of scratch for the tiles' shares of the scale's gradient
 int64_t linear_dx_rbias_dot_floats(const rdb_linear_desc *d) { return cdiv(d->in_f, RB_BI) * cdiv(d->tokens, RB_BT); }
 
+// Ranges of the contraction for tiles of 64 features x 256 tokens (see RB_PART).  A block walks over its contraction alone, 1.06 us per 64
+// values (1.5 with two blocks to a unit), and layers below the sizes of the 256-wide tiles leave units idle meanwhile: 311 tokens x 1432 ->
+// 7936 backward has 46 blocks of 124 stages, 113 us, and 30 in twelve ranges (the sums of which take 8.6); 928 x 1024 -> 6176 94 -> 39; 269 x
+// 2912 -> 632 forward 45 -> 17; 2085 x 1080 -> 2472 backward 46 -> 41.  The model below picks within 5 % of the fastest of 1 to 16 ranges on 24 of
+// 26 layers measured (269 to 5949 tokens, 272 to 7936 features), within 10 % on the others; with tiles enough for the chip, or contractions of less
+// than about 800 values, that is one range (5814 x 272 -> 528: 15.5 us, 20 in two).
+static int64_t rb_tiles(const rdb_linear_desc *d, int64_t cols) { return cdiv(cols, RB_BI) * cdiv(d->tokens, RB_BT); }
+static void rb_ranges(const rdb_linear_desc *d, int64_t cols, int num_cus, int &ranges, int &range_stages)
+{
+    const int64_t tiles = rb_tiles(d, cols), stages = cdiv(cols == d->in_f ? d->out_f : d->in_f, RB_BK);
+    auto per = [&](int r) { return cdiv(cdiv(stages, r), 2) * 2; };   // the main loop takes two stages a turn
+    double best_us = 1e30;
+    ranges = 1;
+    for (int r = 1; r <= 16; ++r) {
+        const int64_t n = per(r);
+        if (r > 1 && (n < 4 || cdiv(stages, n) != r)) continue;
+        const int64_t blocks = tiles * r, rounds = cdiv(blocks, 2 * num_cus);
+        const double us = rounds * (4.0 + n * (blocks > num_cus ? 1.5 : 1.06)) + (r > 1 ? 5.0 + tiles * r * (RB_TILE * 4 * 0.4e-6) : 0.0);
+        if (us < best_us) {
+            best_us = us;
+            ranges = r;
+        }
+    }
+    range_stages = (int)per(ranges);
+}
+// Scratch for the ranges' sums (0: one range), and for one float per block that adds them up
+static int64_t rb_part_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus)
+{
+    int ranges, range_stages;
+    rb_ranges(d, cols, num_cus, ranges, range_stages);
+    return ranges > 1 ? rb_tiles(d, cols) * (ranges * (RB_TILE * 4ll) + RB_BT / 32 * 4ll) : 0;
+}
+
+// What a call uses beyond the tiles' shares of the scale's gradient: R for the 256-wide tiles, or the ranges' sums.
+int64_t rbias_scratch_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus)
+{
+    const int64_t table = rbias_big_table_bytes(d, cols, num_cus);
+    return table > 0 ? table : rb_part_bytes(d, cols, num_cus);
+}
+
 // other / dot_part / dscale: NULL, or the matrix the product is reduced against, room for one float per tile, and where the sum goes;
-// table: NULL, or scratch of table_bytes for R
+// table: NULL, or scratch of table_bytes for R or the ranges' sums
 static int rbias_add(void *dst, int64_t ld_dst, int64_t cols, const void *src, int64_t ld_src, int64_t contraction, uint32_t sR, uint32_t sK,
                      const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, const void *other = nullptr, int64_t ld_other = 0,
-                     float *dot_part = nullptr, float *dscale = nullptr, void *table = nullptr, int64_t table_bytes = 0)
+                     float *dot_part = nullptr, void *dscale = nullptr, int dscale_dtype = RDB_F32, void *table = nullptr, int64_t table_bytes = 0)
 {
     if (d->act_dtype != RDB_BF16 || d->coef_dtype != RDB_BF16 || d->coef_rows == 0 || !scale_bias) return RDB_E_UNSUPPORTED;
     if (d->in_f % 8 || d->out_f % 8 || d->tokens < 1 || d->in_f < 1 || d->out_f < 1) return RDB_E_UNSUPPORTED;
@@ -411,8 +539,24 @@ static int rbias_add(void *dst, int64_t ld_dst, int64_t cols, const void *src, i
                                       num_compute_units(), s))
             return rc;
         if (!other) return RDB_OK;
-        rbias_sum_kernel<<<1, 256, 0, s>>>(dscale, dot_part, tiles);
-        return check_launch("rbias_sum_kernel");
+        return launch_rbias_sum(dscale, dscale_dtype, dot_part, tiles, s);
+    }
+    size_t smem = engine_smem<RB_BI, RB_BT, RB_BK, K_CONT, K_CONT>();
+    const int tiles = p.tiles_i * p.tiles_t;
+    const int64_t part = table && !((uintptr_t)table & 15) ? rb_part_bytes(d, cols, num_compute_units()) : 0;
+    if (part > 0 && table_bytes >= part) {
+        rb_ranges(d, cols, num_compute_units(), p.ranges, p.range_stages);
+        p.part = static_cast<float *>(table);
+        p.dot_part = p.part + (int64_t)tiles * p.ranges * RB_TILE;
+        if (int rc = launch_engine(rbias_add_kernel<RB_PART>, p, tiles * p.ranges, smem, s, "rbias_add_kernel<part>")) return rc;
+        const int blocks = tiles * (RB_BT / 32);
+        if (!other) {
+            rbias_sum_ranges_kernel<false><<<blocks, 256, 0, s>>>(p);
+            return check_launch("rbias_sum_ranges_kernel");
+        }
+        rbias_sum_ranges_kernel<true><<<blocks, 256, 0, s>>>(p);
+        if (int rc = check_launch("rbias_sum_ranges_kernel<dot>")) return rc;
+        return launch_rbias_sum(dscale, dscale_dtype, p.dot_part, blocks, s);
     }
     // tiles of 512 tokens when they give at least every other compute unit a block (half the hashing per product: measured
     // ahead from there on; 8192 tokens x 768 features, contraction 3072: 83 -> 67 us), tiles of 256 tokens otherwise
@@ -430,23 +574,20 @@ static int rbias_add(void *dst, int64_t ld_dst, int64_t cols, const void *src, i
         if (int rl = reserve_lds(reinterpret_cast<const void *>(rbias_wide_kernel<true>), wsmem, "rbias_wide_kernel<dot>")) return rl;
         rbias_wide_kernel<true><<<xcd_grid_size(wide_items), RW_THREADS, wsmem, s>>>(p);
         if (int rc = check_launch("rbias_wide_kernel<dot>")) return rc;
-        rbias_sum_kernel<<<1, 256, 0, s>>>(dscale, dot_part, wide_items);
-        return check_launch("rbias_sum_kernel");
+        return launch_rbias_sum(dscale, dscale_dtype, dot_part, wide_items, s);
     }
-    size_t smem = engine_smem<RB_BI, RB_BT, RB_BK, K_CONT, K_CONT>();
     const size_t stage = (size_t)RB_BT * (RB_BI + 4) * sizeof(float);
     if (smem < stage) smem = stage;
-    if (!other) return launch_engine(rbias_add_kernel<false>, p, p.tiles_i * p.tiles_t, smem, s, "rbias_add_kernel");
-    if (int rc = launch_engine(rbias_add_kernel<true>, p, p.tiles_i * p.tiles_t, smem, s, "rbias_add_kernel<dot>")) return rc;
-    rbias_sum_kernel<<<1, 256, 0, s>>>(dscale, dot_part, p.tiles_i * p.tiles_t);
-    return check_launch("rbias_sum_kernel");
+    if (!other) return launch_engine(rbias_add_kernel<RB_ADD>, p, tiles, smem, s, "rbias_add_kernel");
+    if (int rc = launch_engine(rbias_add_kernel<RB_ADD_DOT>, p, tiles, smem, s, "rbias_add_kernel<dot>")) return rc;
+    return launch_rbias_sum(dscale, dscale_dtype, dot_part, tiles, s);
 }
 
 // dx += s * dy . R and d s = <dy . R, x> in one pass over dy . R
-int linear_dx_rbias_add_dscale(void *dx, int64_t lddx, float *dscale, float *dot_part, const void *dy, int64_t lddy, const void *x, int64_t ldx,
-                               const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table, int64_t table_bytes)
+int linear_dx_rbias_add_dscale(void *dx, int64_t lddx, void *dscale, int dscale_dtype, float *dot_part, const void *dy, int64_t lddy, const void *x,
+                               int64_t ldx, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table, int64_t table_bytes)
 {
-    return rbias_add(dx, lddx, d->in_f, dy, lddy, d->out_f, 1u, (uint32_t)d->in_f, scale_bias, d, s, x, ldx, dot_part, dscale, table, table_bytes);
+    return rbias_add(dx, lddx, d->in_f, dy, lddy, d->out_f, 1u, (uint32_t)d->in_f, scale_bias, d, s, x, ldx, dot_part, dscale, dscale_dtype, table, table_bytes);
 }
 
 // dx += s * dy . R on the launch stream, after the kernels that wrote dx.  Returns RDB_E_UNSUPPORTED (without setting an
@@ -454,14 +595,14 @@ int linear_dx_rbias_add_dscale(void *dx, int64_t lddx, float *dscale, float *dot
 int linear_dx_rbias_add(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table,
                         int64_t table_bytes)
 {
-    return rbias_add(dx, lddx, d->in_f, dy, lddy, d->out_f, 1u, (uint32_t)d->in_f, scale_bias, d, s, nullptr, 0, nullptr, nullptr, table, table_bytes);
+    return rbias_add(dx, lddx, d->in_f, dy, lddy, d->out_f, 1u, (uint32_t)d->in_f, scale_bias, d, s, nullptr, 0, nullptr, nullptr, RDB_F32, table, table_bytes);
 }
 
 // y += s * x . R^T on the launch stream, after the kernels that wrote y; same conditions.
 int linear_fwd_rbias_add(void *y, int64_t ldy, const void *x, int64_t ldx, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table,
                          int64_t table_bytes)
 {
-    return rbias_add(y, ldy, d->out_f, x, ldx, d->in_f, (uint32_t)d->in_f, 1u, scale_bias, d, s, nullptr, 0, nullptr, nullptr, table, table_bytes);
+    return rbias_add(y, ldy, d->out_f, x, ldx, d->in_f, (uint32_t)d->in_f, 1u, scale_bias, d, s, nullptr, 0, nullptr, nullptr, RDB_F32, table, table_bytes);
 }
 
 }  // namespace rdb

@@ -241,6 +241,10 @@ int rdb_linear_project_fwd_rbias(void *y, int64_t ldy, void *state, const void *
 int rdb_linear_rbias_bwd(void *dx, int64_t lddx, float *d_scale_bias, const void *dy, int64_t lddy, const void *x,
                          int64_t ldx, const void *scale_bias, const rdb_linear_desc *desc, void *workspace,
                          int64_t workspace_bytes, void *stream);
+/* rdb_linear_rbias_bwd with the gradient of the scale in fp32 (RDB_F32) or rounded once to bf16 (RDB_BF16). */
+int rdb_linear_rbias_bwd_to(void *dx, int64_t lddx, void *d_scale_bias, int d_scale_bias_dtype, const void *dy, int64_t lddy,
+                            const void *x, int64_t ldx, const void *scale_bias, const rdb_linear_desc *desc, void *workspace,
+                            int64_t workspace_bytes, void *stream);
 
 /* Replaces MmBackward's dW = dy^T x followed by RandumbTensorConstructor.backward ->
  * materialize_bwd (+ scale_bias_bwd) (R.py:979-990): dW is contracted with the regenerated noise tile

@@ -47,6 +47,7 @@ EXPORTS = [
     "rdb_linear_rbias_fwd_ws",
     "rdb_linear_project_fwd_rbias",
     "rdb_linear_rbias_bwd",
+    "rdb_linear_rbias_bwd_to",
     "rdb_linear_bwd_dcoef",
     "rdb_linear_projection_bytes",
     "rdb_linear_projection_preferred",
@@ -183,6 +184,7 @@ def load() -> ctypes.CDLL:
     L.rdb_linear_rbias_fwd_ws.argtypes = [vp, i64, vp, i64, vp, dp, vp, i64, vp]
     L.rdb_linear_project_fwd_rbias.argtypes = [vp, i64, vp, i64, vp, vp, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_rbias_bwd.argtypes = [vp, i64, vp, vp, i64, vp, i64, vp, dp, vp, i64, vp]
+    L.rdb_linear_rbias_bwd_to.argtypes = [vp, i64, vp, ci, vp, i64, vp, i64, vp, dp, vp, i64, vp]
     L.rdb_linear_projection_bytes.argtypes = [dp]
     L.rdb_linear_projection_bytes.restype = i64
     L.rdb_linear_projection_preferred.argtypes = [dp]
@@ -220,7 +222,7 @@ def load() -> ctypes.CDLL:
     L.rdb_selftest_hasty_wait.restype = ci
     for name in ("rdb_sq5_fill_2d", "rdb_sq5_fill_1d", "rdb_materialize_fwd", "rdb_materialize_bwd", "rdb_scale_bias_bwd",
                  "rdb_embed_fwd", "rdb_embed_bwd", "rdb_linear_fwd", "rdb_linear_bwd_dx", "rdb_linear_bwd_dx_dscale", "rdb_linear_rbias_fwd",
-                 "rdb_linear_rbias_fwd_ws", "rdb_linear_project_fwd_rbias", "rdb_linear_rbias_bwd", "rdb_linear_bwd_dcoef",
+                 "rdb_linear_rbias_fwd_ws", "rdb_linear_project_fwd_rbias", "rdb_linear_rbias_bwd", "rdb_linear_rbias_bwd_to", "rdb_linear_bwd_dcoef",
                  "rdb_linear_project", "rdb_linear_project_fwd", "rdb_linear_fwd_projected", "rdb_linear_bwd_dcoef_projected",
                  "rdb_linear_bwd_projected", "rdb_linear_bwd_projected_to", "rdb_linear_bwd_projected_part"):
         getattr(L, name).restype = ci

@@ -747,8 +747,17 @@ extern "C" int rdb_linear_rbias_fwd_ws(void *y, int64_t ldy, const void *x, int6
 extern "C" int rdb_linear_rbias_bwd(void *dx, int64_t lddx, float *d_scale_bias, const void *dy, int64_t lddy, const void *x, int64_t ldx,
                                     const void *scale_bias, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
 {
+    return rdb_linear_rbias_bwd_to(dx, lddx, d_scale_bias, RDB_F32, dy, lddy, x, ldx, scale_bias, d, workspace, workspace_bytes, stream);
+}
+
+extern "C" int rdb_linear_rbias_bwd_to(void *dx, int64_t lddx, void *d_scale_bias, int d_scale_bias_dtype, const void *dy, int64_t lddy, const void *x,
+                                       int64_t ldx, const void *scale_bias, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes,
+                                       void *stream)
+{
     int rc = check_desc("rdb_linear_rbias_bwd", d);
     if (rc) return rc;
+    if (d_scale_bias && d_scale_bias_dtype != RDB_F32 && d_scale_bias_dtype != RDB_BF16)
+        return set_error(RDB_E_DTYPE, "rdb_linear_rbias_bwd: the gradient of the scale leaves as fp32 or bf16, not as dtype %d", d_scale_bias_dtype);
     if (!dx || !dy || !scale_bias) return set_error(RDB_E_NULL, "rdb_linear_rbias_bwd: dx, dy or scale_bias is NULL");
     if (lddx < d->in_f || lddy < d->out_f) return set_error(RDB_E_SHAPE, "rdb_linear_rbias_bwd: leading dimension smaller than the row");
     if ((rc = rbias_request_ok("rdb_linear_rbias_bwd", d))) return rc;
@@ -766,7 +775,8 @@ extern "C" int rdb_linear_rbias_bwd(void *dx, int64_t lddx, float *d_scale_bias,
     const int64_t need = linear_dx_rbias_dot_floats(d) * 4;
     if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 3))
         return set_error(RDB_E_WORKSPACE, "rdb_linear_rbias_bwd: the gradient of the scale needs a workspace of %lld bytes", (long long)need);
-    rc = linear_dx_rbias_add_dscale(dx, lddx, d_scale_bias, RDB_F32, static_cast<float *>(workspace), dy, lddy, x, ldx, scale_bias, d, s, table, room);
+    rc = linear_dx_rbias_add_dscale(dx, lddx, d_scale_bias, d_scale_bias_dtype, static_cast<float *>(workspace), dy, lddy, x, ldx, scale_bias, d, s, table,
+                                    room);
     return rc == RDB_E_UNSUPPORTED ? set_error(RDB_E_UNSUPPORTED, "%s", why) : rc;
 }
 

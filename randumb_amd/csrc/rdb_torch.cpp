@@ -538,9 +538,10 @@ class ProjectedLinear : public Function<ProjectedLinear> {
             const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_BWD_FULL, &r);
             const Tensor ws = bytes(need, dy);
             if (want_sb) {
-                dsb = at::empty({1}, dy.options().dtype(at::kFloat));
-                check(rdb_linear_rbias_bwd(dx.data_ptr(), l.in_f, dsb.data_ptr<float>(), dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), sb.data_ptr(),
-                                           &r, ptr(ws), need, s),
+                const auto dt = scale_bias.scalar_type() == at::kBFloat16 ? at::kBFloat16 : at::kFloat;
+                dsb = at::empty({1}, dy.options().dtype(dt));
+                check(rdb_linear_rbias_bwd_to(dx.data_ptr(), l.in_f, dsb.data_ptr(), code(dt), dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0),
+                                              sb.data_ptr(), &r, ptr(ws), need, s),
                       "rdb_linear_rbias_bwd");
                 dsb = dsb.to(scale_bias.scalar_type());
             } else {

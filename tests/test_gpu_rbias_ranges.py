@@ -42,6 +42,10 @@ def test_ranges_against_float64(T, in_f, out_f):
         assert lib.rdb_linear_rbias_bwd(out.data_ptr(), in_f + 8, d.data_ptr(), dy.data_ptr(), out_f + 8, x.data_ptr(), in_f + 8, s.data_ptr(), ref,
                                         ws.data_ptr(), size, stream) == 0
     assert lib.rdb_linear_rbias_bwd(dx_only.data_ptr(), in_f + 8, None, dy.data_ptr(), out_f + 8, None, 0, s.data_ptr(), ref, ws.data_ptr(), n, stream) == 0
+    ds16 = torch.full((2,), 5.0, dtype=torch.bfloat16, device="cuda")   # the same sum in bf16
+    assert lib.rdb_linear_rbias_bwd_to(dx0.clone().data_ptr(), in_f + 8, ds16.data_ptr(), 1, dy.data_ptr(), out_f + 8, x.data_ptr(), in_f + 8, s.data_ptr(),
+                                       ref, ws.data_ptr(), n, stream) == 0
+    assert torch.equal(ds16, ds.bfloat16())
     assert bool((ws[n:] == 0x5A).all()) and float(ds[1]) == 5.0 and float(ds_one[1]) == 5.0
     assert torch.equal(dx, dx_only)
     for out, old, cols in ((y, y0, out_f), (y_one, y0, out_f), (dx, dx0, in_f), (dx_one, dx0, in_f)):

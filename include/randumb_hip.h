@@ -109,7 +109,7 @@ int64_t rdb_bias_bwd_workspace_bytes(int64_t rows, int64_t n);
  *   out[M x N] = A . B^T (+ bias[N]),  A [M x K], B [N x K] row-major; a_across / b_across: stored transposed, [K x M] / [K x N].
  * out is contiguous.  (0, 0), (0, 1) and (1, 1) of the across flags.  On the bf16 matrix cores at fp32 accuracy (three-way
  * split of both sides, see rdb_set_f32_split; infinities and NaNs as in an fp32 product).  The workspace holds partial sums over ranges
- * of K, added in a fixed order; with less of it (or a bias) fewer ranges run.  RDB_E_UNSUPPORTED: empty, or 2^29 elements or more. */
+ * of K, added in a fixed order; with less of it fewer ranges run.  RDB_E_UNSUPPORTED: empty, or 2^29 elements or more. */
 int rdb_product_f32(float *out, const float *a, int64_t lda, int a_across, const float *b, int64_t ldb, int b_across,
                     const float *bias, int64_t M, int64_t N, int64_t K, void *workspace, int64_t workspace_bytes,
                     void *stream);

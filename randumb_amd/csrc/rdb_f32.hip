@@ -56,13 +56,16 @@ template <typename V> __device__ __forceinline__ V sum_in_order(const float *__r
 }
 
 // out[i] = part[0][i] + part[1][i] + ... in split order, four values per thread (n4 groups of four, then the n % 4 last values
-// one thread each); out fp32, or bf16 (rounded once).  One or two such sums a launch: the second one's blocks follow.
+// one thread each); out fp32, or bf16 (rounded once); bias: NULL, or fp32, added to rows of cols values.  One or two such sums a launch:
+// the second one's blocks follow.
 struct FgSum {
     void *out;
     const float *part;
     int64_t n, stride;   // values, floats between the partial matrices
     int out_bf16, splits, vec;
     int blocks;          // 0: no such sum
+    const float *bias;
+    uint32_t cols;
 };
 __global__ __launch_bounds__(256) void f32_sum_splits_kernel(FgSum a, FgSum b)
 {
@@ -70,12 +73,20 @@ __global__ __launch_bounds__(256) void f32_sum_splits_kernel(FgSum a, FgSum b)
     const FgSum &q = second ? b : a;
     const int64_t i = (int64_t)((int)blockIdx.x - (second ? a.blocks : 0)) * 256 + threadIdx.x, n4 = q.vec ? q.n / 4 : 0;
     if (i < n4) {
-        const f32x4 v = sum_in_order<f32x4>(q.part + i * 4, q.stride, q.splits);
+        f32x4 v = sum_in_order<f32x4>(q.part + i * 4, q.stride, q.splits);
+        if (q.bias) {
+            uint32_t c = (uint32_t)(i * 4) % q.cols;   // n is below 2^29
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[j] += q.bias[c];
+                if (++c == q.cols) c = 0;
+            }
+        }
         if (q.out_bf16) store4<bf16_t>(static_cast<bf16_t *>(q.out) + i * 4, v[0], v[1], v[2], v[3]);
         else *reinterpret_cast<f32x4 *>(static_cast<float *>(q.out) + i * 4) = v;
     } else if (n4 * 4 + (i - n4) < q.n) {
         const int64_t e = n4 * 4 + (i - n4);
-        const float v = sum_in_order<float>(q.part + e, q.stride, q.splits);
+        const float v = sum_in_order<float>(q.part + e, q.stride, q.splits) + (q.bias ? q.bias[(uint32_t)e % q.cols] : 0.0f);
         if (q.out_bf16) static_cast<bf16_t *>(q.out)[e] = f32_to_bf16(v);
         else static_cast<float *>(q.out)[e] = v;
     }
@@ -84,7 +95,7 @@ static FgSum fg_sum(void *out, int out_bf16, const float *part, int64_t n, int64
 {
     if (splits <= 1) return {};
     const int vec = fg_aligned16(out) ? 1 : 0;   // the partial matrices are 256-byte aligned
-    return {out, part, n, stride, out_bf16, splits, vec, (int)cdiv(vec ? n / 4 + n % 4 : n, 256)};
+    return {out, part, n, stride, out_bf16, splits, vec, (int)cdiv(vec ? n / 4 + n % 4 : n, 256), nullptr, 0};
 }
 static int fg_launch_sums(const FgSum &a, const FgSum &b, hipStream_t s)
 {
@@ -159,8 +170,13 @@ template <int ASRC, int BSRC> static int fg_launch_ranges(FgProduct q, int room,
     q.out_bf16 = 0;
     q.kchunk = cdiv(cdiv(q.K, plan.ranges), FG_BK) * FG_BK;   // every range holds something (fg_plan)
     q.split_stride = stride;
+    const float *const bias = q.bias;   // fp32 where there are ranges
+    q.bias = nullptr;
     if (int rc = fg_launch<ASRC, BSRC>(q, num_cus, s, name)) return rc;
-    return fg_launch_sums(fg_sum(out, out_bf16, part, n, stride, plan.ranges), FgSum{}, s);
+    FgSum sum = fg_sum(out, out_bf16, part, n, stride, plan.ranges);
+    sum.bias = bias;
+    sum.cols = (uint32_t)q.N;
+    return fg_launch_sums(sum, FgSum{}, s);
 }
 
 // Two such products that do not need each other, in one launch, and their sums in one: t = dy . C and dC = dy^T . z.
@@ -614,7 +630,7 @@ extern "C" int rdb_product_f32(float *out, const float *a, int64_t lda, int a_ac
                    0, 0, 0, 0, 0u};
     const int64_t stride = up256(M * N * 4);
     int room = product_room(M, N, K, num_cus);
-    if (bias || !workspace || !fg_aligned16(workspace)) room = 1;   // the bias is added by the product's own epilogue
+    if (!workspace || !fg_aligned16(workspace)) room = 1;
     else if (room * stride > workspace_bytes) room = (int)std::max<int64_t>(1, workspace_bytes / stride);
     float *part = static_cast<float *>(workspace);
     hipStream_t s = (hipStream_t)stream;

@@ -91,11 +91,11 @@ __global__ __launch_bounds__(256) void f32_sum_splits_kernel(FgSum a, FgSum b)
         else static_cast<float *>(q.out)[e] = v;
     }
 }
-static FgSum fg_sum(void *out, int out_bf16, const float *part, int64_t n, int64_t stride, int splits)
+static FgSum fg_sum(void *out, int out_bf16, const float *part, int64_t n, int64_t stride, int splits, const float *bias = nullptr, int64_t cols = 0)
 {
-    if (splits <= 1) return {};
+    if (splits <= 1 && !bias) return {};
     const int vec = fg_aligned16(out) ? 1 : 0;   // the partial matrices are 256-byte aligned
-    return {out, part, n, stride, out_bf16, splits, vec, (int)cdiv(vec ? n / 4 + n % 4 : n, 256), nullptr, 0};
+    return {out, part, n, stride, out_bf16, splits, vec, (int)cdiv(vec ? n / 4 + n % 4 : n, 256), bias, (uint32_t)cols};
 }
 static int fg_launch_sums(const FgSum &a, const FgSum &b, hipStream_t s)
 {
@@ -128,8 +128,10 @@ static int fg_es(int dtype) { return dtype == RDB_BF16 ? 2 : 4; }
 // few TFLOP/s, so the factored form on the matrix cores wins also where it is more flops than a product on a stored W.
 static bool fg_wanted(const rdb_linear_desc *) { return true; }
 
-// z = x . N^T and t = dy . C, [tokens x k] over K = in_f or out_f; dC = dy^T . z, [out_f x k] over the tokens: ranges there is room for
-static int zt_room(const rdb_linear_desc *d, int64_t K, int num_cus) { return fg_room(d->tokens, d->k, K, num_cus, 128, 32).ranges; }
+// z = x . N^T and t = dy . C, [tokens x k] over in_f and out_f; dC = dy^T . z, [out_f x k] over the tokens: ranges there is room for.  The
+// two of the backward pass run side by side or alone, with the same sums: short contractions take one range either way.
+static int z_room(const rdb_linear_desc *d, int num_cus) { return fg_room(d->tokens, d->k, d->in_f, num_cus, 128, 32).ranges; }
+static int t_room(const rdb_linear_desc *d, int num_cus) { return fg_room(d->tokens, d->k, d->out_f, num_cus, 128, 32).ranges; }
 static int dc_room(const rdb_linear_desc *d, int num_cus) { return fg_room(d->out_f, d->k, d->tokens, num_cus, 256, 64).ranges; }
 
 // scratch: z or t [tokens x k] and its partial matrices; for the coefficient gradient also one [out_f x k] matrix per token range
@@ -139,13 +141,13 @@ int64_t linear_f32_workspace(int op, const rdb_linear_desc *d, int num_cus)
     if (op == RDB_OP_LINEAR_BWD_DCOEF) dd.coef_dtype = dd.act_dtype;   // reads no coefficients
     if (!fg_ok(&dd)) return 0;
     const int64_t zt = up256(d->tokens * d->k * 4);
-    auto with_parts = [&](int64_t K) { const int r = zt_room(d, K, num_cus); return zt * (r > 1 ? 1 + r : 1); };
-    if (op == RDB_OP_LINEAR_FWD) return with_parts(d->in_f);
-    if (op == RDB_OP_LINEAR_BWD_DX) return with_parts(d->out_f);
+    auto with_parts = [&](int r) { return zt * (r > 1 ? 1 + r : 1); };
+    if (op == RDB_OP_LINEAR_FWD) return with_parts(z_room(d, num_cus));
+    if (op == RDB_OP_LINEAR_BWD_DX) return with_parts(t_room(d, num_cus));
     if (op != RDB_OP_LINEAR_BWD_DCOEF) return 0;
     const int r = dc_room(d, num_cus);
     // ... and, for the gradient of the random bias's scale, one value per 64 x 128 tile of [tokens x out_f]
-    return with_parts(d->in_f) + (r > 1 ? (int64_t)r * up256(d->out_f * d->k * 4) : 0) + up256(cdiv(d->tokens, 64) * cdiv(d->out_f, FG_BN) * 4);
+    return with_parts(z_room(d, num_cus)) + (r > 1 ? (int64_t)r * up256(d->out_f * d->k * 4) : 0) + up256(cdiv(d->tokens, 64) * cdiv(d->out_f, FG_BN) * 4);
 }
 
 static bool fg_ws_ok(int op, const rdb_linear_desc *d, int num_cus, const void *ws, int64_t bytes)
@@ -162,21 +164,22 @@ template <int ASRC, int BSRC> static int fg_launch_ranges(FgProduct q, int room,
     q.groups = plan.groups;
     q.kchunk = 0;
     q.split_stride = 0;
-    if (plan.ranges <= 1) return fg_launch<ASRC, BSRC>(q, num_cus, s, name);
     float *const out = q.out;
+    const float *const bias = q.bias;   // fp32, as out is then
     const int out_bf16 = q.out_bf16;
     const int64_t n = q.M * q.N;
+    if (plan.ranges <= 1) {
+        if (int rc = fg_launch<ASRC, BSRC>(q, num_cus, s, name)) return rc;
+        // the kernels that read a matrix across its rows are not built with a bias: it is added in place
+        return FgGroups<ASRC, BSRC>::biased ? RDB_OK : fg_launch_sums(fg_sum(out, out_bf16, out, n, 0, 1, bias, q.N), FgSum{}, s);
+    }
     q.out = part;
     q.out_bf16 = 0;
     q.kchunk = cdiv(cdiv(q.K, plan.ranges), FG_BK) * FG_BK;   // every range holds something (fg_plan)
     q.split_stride = stride;
-    const float *const bias = q.bias;   // fp32 where there are ranges
     q.bias = nullptr;
     if (int rc = fg_launch<ASRC, BSRC>(q, num_cus, s, name)) return rc;
-    FgSum sum = fg_sum(out, out_bf16, part, n, stride, plan.ranges);
-    sum.bias = bias;
-    sum.cols = (uint32_t)q.N;
-    return fg_launch_sums(sum, FgSum{}, s);
+    return fg_launch_sums(fg_sum(out, out_bf16, part, n, stride, plan.ranges, bias, q.N), FgSum{}, s);
 }
 
 // Two such products that do not need each other, in one launch, and their sums in one: t = dy . C and dC = dy^T . z.
@@ -214,7 +217,7 @@ static int fg_project(float *z, const float *x, int64_t ldx, const rdb_linear_de
     FgProduct q = {x, ldx, (d->tokens - 1) * ldx + d->in_f, nullptr, 0, 0, z, d->k, nullptr, d->tokens, d->k, d->in_f, 0, 0, 0, 0, d->seed};
     q.a_es = fg_es(d->act_dtype);
     const int64_t zt = up256(d->tokens * d->k * 4) / 4;
-    return fg_launch_ranges<FG_KCONT, FG_NOISE_M>(q, std::max(1, std::min(zt_room(d, d->in_f, num_cus), max_ranges)), part ? part : z + zt, zt, num_cus, s, "f32_gemm_kernel (z = x . N^T)");
+    return fg_launch_ranges<FG_KCONT, FG_NOISE_M>(q, std::max(1, std::min(z_room(d, num_cus), max_ranges)), part ? part : z + zt, zt, num_cus, s, "f32_gemm_kernel (z = x . N^T)");
 }
 
 // The three entry points return RDB_E_UNSUPPORTED, without setting an error, when the request does not fit.
@@ -278,7 +281,7 @@ static int fg_backward(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, con
     if (dx && dcoef && f32_split_mode()) {
         float *t = (float *)workspace;
         const int64_t zt = up256(d->tokens * d->k * 4) / 4;
-        if (int rc = fg_launch_pair_ranges(fg_t(t, dy, lddy, coef, d), zt_room(d, d->out_f, num_cus), t + zt, zt, fg_dc(dcoef, dcoef_dtype, dy, lddy, z, d),
+        if (int rc = fg_launch_pair_ranges(fg_t(t, dy, lddy, coef, d), t_room(d, num_cus), t + zt, zt, fg_dc(dcoef, dcoef_dtype, dy, lddy, z, d),
                                            room, dc_part, dc_stride, num_cus, s))
             return rc;
         return fg_dx_from_t(dx, lddx, t, d, num_cus, s);
@@ -298,7 +301,7 @@ int linear_dx_f32(void *dx, int64_t lddx, const void *dy, int64_t lddy, const vo
     float *t = (float *)workspace;
     const int b16 = d->act_dtype == RDB_BF16;
     const int64_t zt = up256(d->tokens * d->k * 4) / 4;
-    if (int rc = fg_launch_ranges<FG_KCONT, FG_MCONT>(fg_t(t, dy, lddy, coef, d), zt_room(d, d->out_f, num_cus), t + zt, zt, num_cus, s, "f32_gemm_kernel (t = dy . C)"))
+    if (int rc = fg_launch_ranges<FG_KCONT, FG_MCONT>(fg_t(t, dy, lddy, coef, d), t_room(d, num_cus), t + zt, zt, num_cus, s, "f32_gemm_kernel (t = dy . C)"))
         return rc;
     if (int rc = fg_dx_from_t(dx, lddx, t, d, num_cus, s)) return rc;
     if (!scale_bias) return RDB_OK;
@@ -323,7 +326,7 @@ int linear_dcoef_f32(float *dcoef, float *d_scale_bias, const void *dy, int64_t 
     if (d->tokens * ldx >= (1ll << 29) || d->tokens * lddy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     float *z = (float *)workspace;
     if (int rc = fg_project(z, (const float *)x, ldx, &dd, num_cus, s)) return rc;
-    const int zs = zt_room(&dd, d->in_f, num_cus);
+    const int zs = z_room(&dd, num_cus);
     float *part = reinterpret_cast<float *>(static_cast<char *>(workspace) + up256(d->tokens * d->k * 4) * (zs > 1 ? 1 + zs : 1));
     const int dcr = dc_room(&dd, num_cus);
     if (int rc = fg_launch_ranges<FG_MCONT, FG_MCONT>(fg_dc(dcoef, RDB_F32, dy, lddy, z, &dd), dcr, part, up256(d->out_f * d->k * 4) / 4, num_cus, s, "f32_gemm_kernel (dC = dy^T . z)")) return rc;

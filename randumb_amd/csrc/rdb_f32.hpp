@@ -721,7 +721,9 @@ inline FgPlan fg_room(int64_t M, int64_t N, int64_t K, int num_cus, int64_t min_
 // file's kinds, [258 .. 7520] x [100 .. 7520] over [100 .. 7520], some 380 plans; what it picks is within 1 % of the best of
 // them on average, 3 % at most): a stage of a group takes `chain` us when it has the compute unit to itself, the groups that
 // share a unit take `unit` us of its throughput each, a launch `base` us and every further round of blocks 2.6; outputs leave at 4.8 TB/s; adding ranges up is one more
-// launch, whose 14 TB/s say that the partial matrices come back out of the caches.  `resident`, the groups that take turns on a unit's
+// launch, whose 14 TB/s say that the partial matrices come back out of the caches.  `host_us`: what that launch counts
+// for besides: a step whose kernels are shorter than the host's work on it (50 to 70 us for a layer) pays for the launch as well, so where the
+// product is short (FG_SHORT_US) ranges have to gain more than both.  `resident`, the groups that take turns on a unit's
 // time, was fitted with the others and is not what registers and LDS leave room for.  The products measured had fp32 matrices; a
 // side that comes from a bf16 matrix takes less LDS and fewer registers (four to seven blocks of 256 threads fit a unit), and hashing
 // is not told apart: for those the constants are what they are for fp32.
@@ -737,7 +739,8 @@ inline int64_t fg_chunk(int64_t K, int r)
     const int64_t chunk = cdiv(cdiv(K, r), FG_BK) * FG_BK;
     return r > 1 && (cdiv(K, chunk) != r || chunk < 64) ? 0 : chunk;
 }
-inline FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int max_ranges, bool groups4)
+constexpr double FG_HOST_US = 3.8, FG_SHORT_US = 16.0;
+inline FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int max_ranges, bool groups4, double host_us = 0.0)
 {
     const bool split = f32_split_mode() != 0;
     const double out_mb = (double)M * N * 4e-6;
@@ -751,8 +754,9 @@ inline FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int max_rang
             if (!chunk) continue;
             const int64_t per_cu = cdiv(tiles * r, num_cus), stages = cdiv(chunk / FG_BK, kd.groups);
             const int64_t rounds = cdiv(per_cu, kd.resident);
-            const double us = kd.base + 2.6 * (rounds - 1) + stages * (rounds * kd.chain + per_cu * kd.groups * kd.unit) + out_mb * r * 0.21 +
+            double us = kd.base + 2.6 * (rounds - 1) + stages * (rounds * kd.chain + per_cu * kd.groups * kd.unit) + out_mb * r * 0.21 +
                               (r > 1 ? 4.2 + out_mb * r * 0.07 : 0.0);
+            if (r > 1 && us < FG_SHORT_US) us += host_us;
             if (us < best_us) {
                 best_us = us;
                 best = {kd.bm, r, kd.groups};

@@ -753,7 +753,7 @@ extern "C" int rdb_embed_bwd(float *dcoef, const int64_t *idx, int64_t n_idx, co
 // ----------------------------------------------------------------------------------------------- gradient of a pseudorandom bias
 // b[o] = sum_m noise(PRIME*o + m) coef[m] + s noise1d(o), added to every row of y: with g[o] = sum_t dy[t, o],
 // dcoef[m] = sum_o g[o] noise(PRIME*o + m) and ds = sum_o g[o] noise1d(o).
-// First launch: the column sums of dy, a chunk of rows per block (memory-bound: dy is read once, 16 bytes a lane where its rows
+// A small dy: one launch (bias_grad_direct_kernel).  Otherwise two.  First launch: the column sums of dy, a chunk of rows per block (memory-bound: dy is read once, 16 bytes a lane where its rows
 // allow), partial sums [chunks x n].  Second launch: every block adds the chunks up again for itself (a few rows out of L2)
 // and contracts them with the noise of its own BIAS_M coefficients; the n * k hashes are few.  Fixed orders throughout.
 // Replaces a column sum by the library, its cast, the contraction and the sum over its splits: 128 tokens x 256, k = 64: 12.6 ->
@@ -809,32 +809,21 @@ template <typename T, int V> __global__ __launch_bounds__(NT) void column_sums_k
     }
 }
 
-// block b: coefficients b * BIAS_M .. + 3; the block behind the last coefficient: the scale.  THREADS: a thread's outputs are a chain of
-// memory latencies, so long biases take blocks of 1024 (3072 outputs, k = 256: 15.7 us with 256 threads, 12 turns of the loop; vector-coef layer step 561 -> 540).
-template <int THREADS> __global__ __launch_bounds__(THREADS) void bias_grad_kernel(float *__restrict__ dcoef, float *__restrict__ ds, const float *__restrict__ part, int chunks, int64_t n, int64_t k,
-                                                       uint32_t seed)
+// What a block of the gradient does with a column's sum g (block b: coefficients b * BIAS_M .. + 3; the block behind the last
+// coefficient: the scale), and at the end with its threads' shares.
+__device__ __forceinline__ void bias_contract(float (&acc)[BIAS_M], float g, uint32_t o, int64_t m0, bool scale, uint32_t seed)
+{
+    if (scale) {
+        acc[0] = fmaf(g, noise1d(o, seed), acc[0]);
+    } else {
+        const uint32_t f = sq5_first(o, (uint32_t)m0, seed);
+#pragma unroll
+        for (int j = 0; j < BIAS_M; ++j) acc[j] = fmaf(g, sq5_unit(sq5_tail(f + (uint32_t)j * SQ5_N1)), acc[j]);
+    }
+}
+template <int THREADS> __device__ __forceinline__ void bias_finish(float (&acc)[BIAS_M], float *dcoef, float *ds, int64_t m0, int64_t k, bool scale)
 {
     __shared__ float sh[BIAS_M][THREADS / 64];
-    const int64_t m0 = (int64_t)blockIdx.x * BIAS_M;
-    const bool scale = !dcoef || m0 >= k;
-    float acc[BIAS_M] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int64_t o = threadIdx.x; o < n; o += THREADS) {
-        float g = 0.0f;
-        for (int c0 = 0; c0 < chunks; c0 += 8) {   // eight loads in flight
-            float v[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = part[(int64_t)(c0 + i < chunks ? c0 + i : chunks - 1) * n + o];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) g += c0 + i < chunks ? v[i] : 0.0f;
-        }
-        if (scale) {
-            acc[0] = fmaf(g, noise1d((uint32_t)o, seed), acc[0]);
-        } else {
-            const uint32_t f = sq5_first((uint32_t)o, (uint32_t)m0, seed);
-#pragma unroll
-            for (int j = 0; j < BIAS_M; ++j) acc[j] = fmaf(g, sq5_unit(sq5_tail(f + (uint32_t)j * SQ5_N1)), acc[j]);
-        }
-    }
 #pragma unroll
     for (int j = 0; j < BIAS_M; ++j) {
 #pragma unroll
@@ -854,6 +843,61 @@ template <int THREADS> __global__ __launch_bounds__(THREADS) void bias_grad_kern
     }
 }
 
+// The whole gradient in one launch, for a dy so small that every block may read it: blocks of 1024 threads, as many of them side by side
+// on a column's rows as its outputs leave room for, sixteen rows in flight each.  3.3 us and 1.3 for every sixteen rows of a thread, against
+// 8.2 (and a launch more on the host) for the two: 128 rows x 256 5.9, 128 x 10 4.6, 512 x 128 8.5; 250 x 262, six turns, 11.0.
+constexpr int64_t BIAS_DIRECT_BYTES = 256 << 10, BIAS_DIRECT_TURNS = 4;
+constexpr int BIAS_AHEAD = 16;
+static int bias_wide(int64_t n) { return n < 1024 ? (int)cdiv(n, 64) * 64 : 1024; }   // threads along the outputs
+static bool bias_direct(int64_t rows, int64_t n, int es)
+{
+    if (rows <= 0 || n <= 0 || rows * n * es > BIAS_DIRECT_BYTES) return false;
+    const int wide = bias_wide(n);
+    return cdiv(rows, BIAS_AHEAD * (1024 / wide)) * cdiv(n, wide) <= BIAS_DIRECT_TURNS;
+}
+template <typename T> __global__ __launch_bounds__(1024) void bias_grad_direct_kernel(float *__restrict__ dcoef, float *__restrict__ ds, const T *__restrict__ dy,
+                                                                                     int64_t ldy, int rows, int n, int wide, int64_t k, uint32_t seed)
+{
+    const int64_t m0 = (int64_t)blockIdx.x * BIAS_M;
+    const bool scale = !dcoef || m0 >= k;
+    const int beside = 1024 / wide, first = (int)threadIdx.x / wide;
+    float acc[BIAS_M] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int o = (int)threadIdx.x - first * wide; o < n && first < beside; o += wide) {
+        float g = 0.0f;
+        for (int r0 = first; r0 < rows; r0 += BIAS_AHEAD * beside) {
+            float v[BIAS_AHEAD];
+#pragma unroll
+            for (int i = 0; i < BIAS_AHEAD; ++i) v[i] = to_f32(dy[(int64_t)min(r0 + i * beside, rows - 1) * ldy + o]);   // clamped: loaded, not added
+#pragma unroll
+            for (int i = 0; i < BIAS_AHEAD; ++i) g += r0 + i * beside < rows ? v[i] : 0.0f;
+        }
+        bias_contract(acc, g, (uint32_t)o, m0, scale, seed);
+    }
+    bias_finish<1024>(acc, dcoef, ds, m0, k, scale);
+}
+
+// The second launch.  THREADS: a thread's outputs are a chain of
+// memory latencies, so long biases take blocks of 1024 (3072 outputs, k = 256: 15.7 us with 256 threads, 12 turns of the loop; vector-coef layer step 561 -> 540).
+template <int THREADS> __global__ __launch_bounds__(THREADS) void bias_grad_kernel(float *__restrict__ dcoef, float *__restrict__ ds, const float *__restrict__ part, int chunks, int64_t n, int64_t k,
+                                                       uint32_t seed)
+{
+    const int64_t m0 = (int64_t)blockIdx.x * BIAS_M;
+    const bool scale = !dcoef || m0 >= k;
+    float acc[BIAS_M] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int64_t o = threadIdx.x; o < n; o += THREADS) {
+        float g = 0.0f;
+        for (int c0 = 0; c0 < chunks; c0 += 8) {   // eight loads in flight
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = part[(int64_t)(c0 + i < chunks ? c0 + i : chunks - 1) * n + o];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) g += c0 + i < chunks ? v[i] : 0.0f;
+        }
+        bias_contract(acc, g, (uint32_t)o, m0, scale, seed);
+    }
+    bias_finish<THREADS>(acc, dcoef, ds, m0, k, scale);
+}
+
 }  // namespace rdb
 
 extern "C" int64_t rdb_bias_bwd_workspace_bytes(int64_t rows, int64_t n) { return rows >= 0 && n > 0 ? bias_chunks(rows) * n * (int64_t)sizeof(float) : 0; }
@@ -870,6 +914,13 @@ extern "C" int rdb_bias_bwd(float *dcoef, float *ds, const void *dy, int dtype, 
     hipStream_t s = (hipStream_t)stream;
     float *part = static_cast<float *>(workspace);
     int chunks = bias_chunks(rows);
+    const int64_t blocks = (dcoef ? cdiv(k, BIAS_M) : 0) + (ds ? 1 : 0);
+    if (bias_direct(rows, n, dtype == RDB_BF16 ? 2 : 4)) {
+        const int wide = bias_wide(n);
+        if (dtype == RDB_BF16) bias_grad_direct_kernel<bf16_t><<<(unsigned)blocks, 1024, 0, s>>>(dcoef, ds, static_cast<const bf16_t *>(dy), ldy, (int)rows, (int)n, wide, k, seed);
+        else bias_grad_direct_kernel<float><<<(unsigned)blocks, 1024, 0, s>>>(dcoef, ds, static_cast<const float *>(dy), ldy, (int)rows, (int)n, wide, k, seed);
+        return check_launch("bias_grad_direct_kernel");
+    }
     if (n > 0) {
         if (!workspace || ((uintptr_t)workspace & 3) || workspace_bytes < rdb_bias_bwd_workspace_bytes(rows, n))
             return set_error(RDB_E_WORKSPACE, "rdb_bias_bwd: workspace of %lld bytes needed, %lld given", (long long)rdb_bias_bwd_workspace_bytes(rows, n),
@@ -887,7 +938,6 @@ extern "C" int rdb_bias_bwd(float *dcoef, float *ds, const void *dy, int dtype, 
         }
         if (int rc = check_launch("column_sums_kernel")) return rc;
     }
-    const int64_t blocks = (dcoef ? cdiv(k, BIAS_M) : 0) + (ds ? 1 : 0);
     if (n > 512) bias_grad_kernel<1024><<<(unsigned)blocks, 1024, 0, s>>>(dcoef, ds, part, chunks, n, k, seed);
     else bias_grad_kernel<NT><<<(unsigned)blocks, NT, 0, s>>>(dcoef, ds, part, chunks, n, k, seed);
     return check_launch("bias_grad_kernel");

@@ -1,0 +1,32 @@
+"""Gradient of a pseudorandom bias: a dy small enough for one launch, and the sizes around the line to two."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# one output, one row, as many threads side by side as there are, none beside, outputs past one turn of the block, just past the line
+@pytest.mark.parametrize("rows,n,k", [(1, 1, 1), (128, 10, 64), (17, 64, 5), (511, 65, 33), (64, 1000, 16), (33, 1025, 7), (1, 4097, 3), (64, 1024, 8), (65, 1024, 8)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_against_float64(rows, n, k, dtype):
+    from randumb_amd import _lib, hip
+
+    print(f"case bias gradient {rows} x {n} k={k} {dtype}", flush=True)
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator().manual_seed(rows + n + k)
+    wide = torch.randn(rows, n + 3, generator=g).to(dtype).cuda()   # rows with a leading dimension
+    dy = wide[:, :n]
+    need = lib.rdb_bias_bwd_workspace_bytes(rows, n)
+    ws = torch.full((need + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+    dc, ds = torch.full((k + 1,), 7.0, device="cuda"), torch.full((2,), 7.0, device="cuda")
+    call = lambda c, s: lib.rdb_bias_bwd(c, s, dy.data_ptr(), int(dtype == torch.bfloat16), n + 3, rows, n, k, 11, ws.data_ptr(), need, stream)
+    assert call(dc.data_ptr(), ds.data_ptr()) == 0
+    sums = dy.double().sum(0)
+    noise, line = hip.sq5_fill_2d(n, k, 11).double(), hip.sq5_fill_1d(n, 11).double()
+    # fp32 sums of rows * n terms: 2^-24 sqrt(rows * n) of their root sum of squares
+    bound = 1.2e-7 * (rows * n) ** 0.5 * float(dy.double().norm()) + 1e-6
+    assert float((dc[:k].double() - sums @ noise).abs().max()) < bound and abs(float(ds[0]) - float(sums @ line)) < bound
+    assert float(dc[k]) == 7.0 and float(ds[1]) == 7.0 and bool((ws[need:] == 0x5A).all())
+    alone = [t.clone() for t in (dc, ds)]
+    assert call(alone[0].data_ptr(), 0) == 0 and call(0, alone[1].data_ptr()) == 0
+    assert torch.equal(alone[0], dc) and torch.equal(alone[1], ds)

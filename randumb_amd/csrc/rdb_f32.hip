@@ -130,7 +130,10 @@ static bool fg_wanted(const rdb_linear_desc *) { return true; }
 
 // z = x . N^T and t = dy . C, [tokens x k] over in_f and out_f; dC = dy^T . z, [out_f x k] over the tokens: ranges there is room for.  The
 // two of the backward pass run side by side or alone, with the same sums: short contractions take one range either way.
-static int z_room(const rdb_linear_desc *d, int num_cus) { return fg_room(d->tokens, d->k, d->in_f, num_cus, 64, 32).ranges; }
+static int z_room(const rdb_linear_desc *d, int num_cus)
+{
+    return fg_room(d->tokens, d->k, d->in_f, num_cus, d->tokens < 32 ? 128 : 64, 32).ranges;   // fewer tokens: only what rdb_few.hip leaves
+}
 static int t_room(const rdb_linear_desc *d, int num_cus) { return fg_room(d->tokens, d->k, d->out_f, num_cus, 128, 32).ranges; }
 static int dc_room(const rdb_linear_desc *d, int num_cus) { return fg_room(d->out_f, d->k, d->tokens, num_cus, 256, 64).ranges; }
 
@@ -213,10 +216,11 @@ static int fg_launch_pair_ranges(FgProduct t, int t_room, float *t_part, int64_t
 // z[T x k] = src[T x in_f] . N^T; the partial matrices of its ranges go to `part` (room for max_ranges of them, up256(T k 4)
 // bytes apart; NULL: right behind z, as many as there is room for)
 static int fg_project(float *z, const float *x, int64_t ldx, const rdb_linear_desc *d, int num_cus, hipStream_t s, float *part = nullptr,
-                      int max_ranges = 1 << 30)
+                      int max_ranges = 1 << 30, const FgValues &values = {})
 {
     FgProduct q = {x, ldx, (d->tokens - 1) * ldx + d->in_f, nullptr, 0, 0, z, d->k, nullptr, d->tokens, d->k, d->in_f, 0, 0, 0, 0, d->seed};
     q.a_es = fg_es(d->act_dtype);
+    q.values = values;
     const int64_t zt = up256(d->tokens * d->k * 4) / 4;
     return fg_launch_ranges<FG_KCONT, FG_NOISE_M>(q, std::max(1, std::min(z_room(d, num_cus), max_ranges)), part ? part : z + zt, zt, num_cus, s,
                                                   "f32_gemm_kernel (z = x . N^T)", FG_HOST_US);
@@ -394,15 +398,21 @@ static int fg_rbias(FgProduct q, const void *scale, const rdb_linear_desc *d, in
     return fg_launch<FG_KCONT, FG_NOISE_1D>(q, num_cus, s, name);
 }
 
+// values: NULL, or a pseudorandom bias whose values the launch of the projection forms on the side (an fp32 layer's; then `bias`)
 int linear_fwd_kept_f32(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
-                        const rdb_linear_desc *d, int num_cus, hipStream_t s)
+                        const rdb_pseudo_bias *values, const rdb_linear_desc *d, int num_cus, hipStream_t s)
 {
+    FgValues v = {};
+    if (values) {
+        v = {values->values, values->coef, values->scale, (int)d->out_f, (int)values->k, values->seed};
+        bias = values->values;
+    }
     if (!linear_kept_f32_bytes(d) || !fg_aligned16(kept) || d->tokens * ldx >= (1ll << 29) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     float *z = static_cast<float *>(kept);
     // the partial matrices of the projection's ranges lie in y's memory, which is written last
     const bool room = ldy == d->out_f && fg_aligned16(y);
     const int max_ranges = room ? (int)std::min<int64_t>(32, d->tokens * d->out_f * fg_es(d->act_dtype) / up256(d->tokens * d->k * 4)) : 1;
-    if (int rc = fg_project(z, (const float *)x, ldx, d, num_cus, s, room ? (float *)y : z, max_ranges)) return rc;
+    if (int rc = fg_project(z, (const float *)x, ldx, d, num_cus, s, room ? (float *)y : z, max_ranges, v)) return rc;
     FgProduct q = {z, d->k, d->tokens * d->k, (const float *)coef, d->k, d->out_f * d->k, (float *)y, ldy, (const float *)bias, d->tokens, d->out_f, d->k,
                    0, 0, 0, 0, d->seed};
     q.b_es = fg_es(d->coef_dtype);

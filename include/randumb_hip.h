@@ -59,6 +59,15 @@ int rdb_sq5_fill_2d(float *out, int64_t N, int64_t M, uint32_t seed, void *strea
 /* Replace: squirrel5_generate_1d / squirrel5_kernel_1d (R.py:108-126).  out[n] = noise(n, seed). */
 int rdb_sq5_fill_1d(float *out, int64_t N, uint32_t seed, void *stream);
 
+/* A pseudorandom bias in fp32, b[o] = sum_m noise(PRIME*o + m) coef[m] (+ scale[0] noise1d(o)), and where its values go. */
+typedef struct rdb_pseudo_bias {
+    const float *coef;    /* k values */
+    const float *scale;   /* NULL, or one value */
+    float *values;        /* out_f values */
+    int64_t k;
+    uint32_t seed;
+} rdb_pseudo_bias;
+
 /* ------------------------------------------------------------------------------------------ materialise
  * Replaces: op rten::materialize_fwd + materialize_fwd_kernel (R.py:235-290, 371-381) and
  * rten_cpp::materialize_fwd (R.cpp:38, R.cu:74-152).
@@ -72,6 +81,11 @@ int rdb_sq5_fill_1d(float *out, int64_t N, uint32_t seed, void *stream);
 int rdb_materialize_fwd(float *out, const void *coef, int coef_dtype, int64_t coef_rows, int64_t k,
                         int64_t row_len, int64_t P, int64_t Q, int64_t sP, int64_t sQ, uint32_t seed,
                         const void *scale_bias, void *stream);
+
+/* The weight (n values, contiguous) and the bias (bias_n values) of a vector-coef layer in fp32: what two calls of rdb_materialize_fwd
+ * write, in one launch where the weight is small. */
+int rdb_materialize_weight_and_bias(float *weight, int64_t n, const float *coef, int64_t k, uint32_t seed, const float *scale,
+                                    const rdb_pseudo_bias *bias, int64_t bias_n, void *stream);
 
 /* Replaces: op rten::materialize_bwd + materialize_bwd_kernel (R.py:304-359, 383-390).
  * dW is a contiguous tensor of Nw elements (dtype dw_dtype).  dcoef is fp32 and is OVERWRITTEN:
@@ -365,6 +379,10 @@ int rdb_linear_bwd_projected_to(void *dx, int64_t lddx, void *dcoef, int dcoef_d
 int64_t rdb_linear_kept_bytes(const rdb_linear_desc *desc);
 int rdb_linear_fwd_kept(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef,
                         const void *scale_bias, const void *bias, const rdb_linear_desc *desc, void *stream);
+/* The same for an fp32 layer with a pseudorandom bias, b[o] = sum_m noise(PRIME*o + m) coef[m] (+ scale[0] noise1d(o)): its values (out_f
+ * floats, overwritten) are formed beside the projection, in the same launch.  RDB_E_UNSUPPORTED: another dtype, k or out_f of 2^31 or more. */
+int rdb_linear_fwd_kept_pseudo_bias(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef,
+                                    const void *scale_bias, const rdb_pseudo_bias *bias, const rdb_linear_desc *desc, void *stream);
 int rdb_linear_bwd_kept(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy,
                         int64_t lddy, const void *x, int64_t ldx, const void *kept, const void *coef,
                         const void *scale_bias, const rdb_linear_desc *desc, void *workspace, int64_t workspace_bytes,

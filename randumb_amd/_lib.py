@@ -26,6 +26,7 @@ EXPORTS = [
     "rdb_sq5_fill_2d",
     "rdb_sq5_fill_1d",
     "rdb_materialize_fwd",
+    "rdb_materialize_weight_and_bias",
     "rdb_materialize_bwd",
     "rdb_materialize_bwd_workspace_bytes",
     "rdb_scale_bias_bwd",
@@ -62,6 +63,7 @@ EXPORTS = [
     "rdb_linear_bwd_projected_part",
     "rdb_linear_kept_bytes",
     "rdb_linear_fwd_kept",
+    "rdb_linear_fwd_kept_pseudo_bias",
     "rdb_linear_bwd_kept",
     "rdb_set_big_tiles",
     "rdb_set_f32_split",
@@ -150,6 +152,8 @@ def load() -> ctypes.CDLL:
     L.rdb_last_error_string.argtypes = []
     L.rdb_sq5_fill_2d.argtypes = [vp, i64, i64, u32, vp]
     L.rdb_sq5_fill_1d.argtypes = [vp, i64, u32, vp]
+    L.rdb_materialize_weight_and_bias.argtypes = [vp, i64, vp, i64, u32, vp, vp, i64, vp]
+    L.rdb_materialize_weight_and_bias.restype = ci
     L.rdb_materialize_fwd.argtypes = [vp, vp, ci, i64, i64, i64, i64, i64, i64, i64, u32, vp, vp]
     L.rdb_materialize_bwd.argtypes = [vp, vp, ci, i64, i64, i64, i64, u32, vp, i64, vp]
     L.rdb_materialize_bwd_workspace_bytes.argtypes = [i64, i64, i64, i64]
@@ -204,6 +208,8 @@ def load() -> ctypes.CDLL:
     L.rdb_linear_kept_bytes.restype = i64
     L.rdb_linear_fwd_kept.argtypes = [vp, i64, vp, vp, i64, vp, vp, vp, dp, vp]
     L.rdb_linear_fwd_kept.restype = ci
+    L.rdb_linear_fwd_kept_pseudo_bias.argtypes = [vp, i64, vp, vp, i64, vp, vp, vp, dp, vp]
+    L.rdb_linear_fwd_kept_pseudo_bias.restype = ci
     L.rdb_linear_bwd_kept.argtypes = [vp, i64, vp, ci, vp, vp, i64, vp, i64, vp, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_bwd_kept.restype = ci
     L.rdb_set_big_tiles.argtypes = [ci]

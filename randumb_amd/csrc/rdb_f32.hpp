@@ -30,6 +30,31 @@ enum FgEpilogue {
     FG_STORE_RBIAS = 4  // out = acc + scale[0] * noise1d(row * nsR + column * nsK): materialising W = C . N + s . R
 };
 
+// Values of a contiguous vector-coef tensor in fp32, by blocks of their own beside a product's: out[e] = sum_m noise(e, m) coef[m] (+ scale[0]
+// noise1d(e)), sixteen lanes an element, added up as the kernel that forms such tensors does.
+struct FgValues {
+    float *out;
+    const float *coef, *scale;   // scale: NULL, or one value
+    int n, k;                    // n: 0: no such blocks
+    uint32_t seed;
+};
+__device__ __forceinline__ void fg_values(const FgValues &v, int thread, int threads)
+{
+    constexpr int LANES = 16;
+    const int part = thread % LANES;
+    for (int e = thread / LANES; e < v.n; e += threads / LANES) {
+        uint32_t first = sq5_first((uint32_t)e, (uint32_t)part, v.seed);
+        float acc = 0.0f;
+        for (int m = part; m < v.k; m += LANES) {
+            acc = fmaf(sq5_unit(sq5_tail(first)), v.coef[m], acc);
+            first += LANES * SQ5_N1;
+        }
+#pragma unroll
+        for (int w = 1; w < LANES; w *= 2) acc += __shfl_xor(acc, w);
+        if (part == 0) v.out[e] = v.scale ? acc + v.scale[0] * noise1d((uint32_t)e, v.seed) : acc;
+    }
+}
+
 struct FgParams {
     const float *a;   // A operand's matrix (FG_KCONT / FG_MCONT)
     int64_t lda;
@@ -50,6 +75,7 @@ struct FgParams {
     const float *dotm;          // FG_DOT, FG_ADD_SCALED (or NULL): [M x N] matrix, leading dimension lddot
     int64_t lddot;
     float *dot_part;            // with dotm: one value per block, in block order (x fastest, then y)
+    FgValues values;            // FG_NOISE_M on the B side: formed by the last blocks along z
 };
 
 // fp32 products on the bf16 matrix cores.  v = h + m + l exactly, each part a bf16: v rounded to the nearest, what is left rounded to
@@ -684,6 +710,13 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
 {
     __shared__ __align__(16) float lds[FgBlock<BM, G, ASRC, BSRC, VEC, SPLIT, AES, BES>::LDS];
     __shared__ int not_finite;   // some thread's sum is an infinity or a NaN
+    if constexpr (BSRC == FG_NOISE_M) {
+        if (p.values.n && blockIdx.z == gridDim.z - 1) {
+            constexpr int THREADS = FG_THREADS * G;
+            fg_values(p.values, (int)(blockIdx.y * gridDim.x + blockIdx.x) * THREADS + (int)threadIdx.x, (int)(gridDim.x * gridDim.y) * THREADS);
+            return;
+        }
+    }
     f32_gemm_block<BM, G, ASRC, BSRC, EPI, VEC, SPLIT, AES, BES>(p, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, lds, not_finite);
 }
 
@@ -846,6 +879,7 @@ struct FgProduct {
     // the products as six bf16 matrix instructions on three-way splits of the operands (fg_split3); materialising stays on the
     // fp32 matrix instructions (its unit-coefficient results are compared bit for bit)
     bool split = f32_split_mode() != 0;
+    FgValues values = {};
 };
 
 #define FG_LAUNCH_GROUPS(BM_, G_, EPI_)                                                                               \
@@ -916,6 +950,7 @@ inline FgParams fg_params(const FgProduct &q)
     p.dotm = q.dotm;
     p.lddot = q.lddot;
     p.dot_part = q.dot_part;
+    p.values = q.values;
     return p;
 }
 // 16-byte pieces (8 of a bf16 matrix: four values) when both matrices allow them: aligned bases and leading dimensions, and the extent
@@ -942,7 +977,7 @@ template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_
     const bool vec = fg_vec(q, ASRC, BSRC);
     const bool a16 = (ASRC == FG_KCONT || ASRC == FG_MCONT) && q.a_es == 2, b16 = (BSRC == FG_KCONT || BSRC == FG_MCONT) && q.b_es == 2;
     if (q.split && ((a16 && b16) ? !Groups::a16_b16 : a16 ? !Groups::a16_b32 : b16 && !Groups::a32_b16)) return RDB_E_UNSUPPORTED;
-    const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)splits);
+    const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)(splits + (BSRC == FG_NOISE_M && q.values.n ? 1 : 0)));
     auto run = [&](auto epi_) {
         constexpr int EPI = decltype(epi_)::value;
         if (q.bm == 128 && q.groups == 2) FG_LAUNCH_GROUPS(128, 2, EPI);

@@ -1285,7 +1285,7 @@ extern "C" int rdb_linear_bwd_projected_to(void *dx, int64_t lddx, void *dcoef, 
 // ----------------------------------------------------------------------------------------------- z kept from forward to backward
 namespace rdb {   // rdb_f32.hip
 int64_t linear_kept_f32_bytes(const rdb_linear_desc *d);
-int linear_fwd_kept_f32(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
+int linear_fwd_kept_f32(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias, const rdb_pseudo_bias *values,
                         const rdb_linear_desc *d, int num_cus, hipStream_t s);
 int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x, int64_t ldx,
                         const void *kept, const void *coef, const void *scale_bias, const rdb_linear_desc *d, int num_cus, void *workspace,
@@ -1298,15 +1298,34 @@ extern "C" int64_t rdb_linear_kept_bytes(const rdb_linear_desc *d)
     return linear_kept_f32_bytes(d);
 }
 
+static int fwd_kept(const char *who, void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
+                    const rdb_pseudo_bias *values, const rdb_linear_desc *d, void *stream)
+{
+    if (int rc = check_desc(who, d)) return rc;
+    if (!rdb_linear_kept_bytes(d)) return set_error(RDB_E_UNSUPPORTED, "%s: a layer of which nothing is kept (rdb_linear_kept_bytes)", who);
+    if (!y || !kept || !x || !coef) return set_error(RDB_E_NULL, "%s: y, kept, x or coef is NULL", who);
+    if (ldx < d->in_f || ldy < d->out_f) return set_error(RDB_E_SHAPE, "%s: leading dimension smaller than the row", who);
+    if (values) {
+        if (!values->values || (!values->coef && values->k > 0)) return set_error(RDB_E_NULL, "%s: the bias's coef or values is NULL", who);
+        if (values->k < 0) return set_error(RDB_E_SHAPE, "%s: a bias of %lld coefficients", who, (long long)values->k);
+        if (d->act_dtype != RDB_F32 || values->k >= (1ll << 31) || d->out_f >= (1ll << 31))
+            return set_error(RDB_E_UNSUPPORTED, "%s: fp32 layers, fewer than 2^31 coefficients and outputs", who);
+    }
+    const int rc = linear_fwd_kept_f32(y, ldy, kept, x, ldx, coef, scale_bias, bias, values, d, num_compute_units(), (hipStream_t)stream);
+    return rc == RDB_E_UNSUPPORTED ? set_error(rc, "%s: kept must be 16-byte aligned and tokens * ldx, tokens * ldy below 2^29", who) : rc;
+}
+
 extern "C" int rdb_linear_fwd_kept(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
                                    const rdb_linear_desc *d, void *stream)
 {
-    if (int rc = check_desc("rdb_linear_fwd_kept", d)) return rc;
-    if (!rdb_linear_kept_bytes(d)) return set_error(RDB_E_UNSUPPORTED, "rdb_linear_fwd_kept: a layer of which nothing is kept (rdb_linear_kept_bytes)");
-    if (!y || !kept || !x || !coef) return set_error(RDB_E_NULL, "rdb_linear_fwd_kept: y, kept, x or coef is NULL");
-    if (ldx < d->in_f || ldy < d->out_f) return set_error(RDB_E_SHAPE, "rdb_linear_fwd_kept: leading dimension smaller than the row");
-    const int rc = linear_fwd_kept_f32(y, ldy, kept, x, ldx, coef, scale_bias, bias, d, num_compute_units(), (hipStream_t)stream);
-    return rc == RDB_E_UNSUPPORTED ? set_error(rc, "rdb_linear_fwd_kept: kept must be 16-byte aligned and tokens * ldx, tokens * ldy below 2^29") : rc;
+    return fwd_kept("rdb_linear_fwd_kept", y, ldy, kept, x, ldx, coef, scale_bias, bias, nullptr, d, stream);
+}
+
+extern "C" int rdb_linear_fwd_kept_pseudo_bias(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias,
+                                               const rdb_pseudo_bias *bias, const rdb_linear_desc *d, void *stream)
+{
+    if (!bias) return set_error(RDB_E_NULL, "rdb_linear_fwd_kept_pseudo_bias: bias is NULL");
+    return fwd_kept("rdb_linear_fwd_kept_pseudo_bias", y, ldy, kept, x, ldx, coef, scale_bias, nullptr, bias, d, stream);
 }
 
 extern "C" int rdb_linear_bwd_kept(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x,

@@ -62,6 +62,7 @@ constexpr int COEF_CHUNK = 2048;
 constexpr float MAT_LARGE = 3.777893186295716e22f;   // 2^75
 constexpr int MAT_UNROLL = 8;
 constexpr int MAT_SHORT = 48;
+constexpr int64_t MAT_PAIR_HASHES = (int64_t)1 << 27;   // a weight and its bias in one launch: up to some 45 us of hashing
 
 struct MatVecParams {
     float *out;
@@ -75,10 +76,9 @@ struct MatVecParams {
 // LANES > 1: that many neighbouring lanes share an element, lane l its terms l, l + LANES, .. (then added up across the lanes, nearest
 // first): with few elements the chip is not full, and the chain's length is what a launch takes (3072 elements, k = 256: 16.5 ->
 // 4 us).  SHORT: at most MAT_SHORT terms.
-template <bool GATHER, int LANES, bool SHORT> __global__ __launch_bounds__(NT) void materialize_vec_kernel(MatVecParams p)
+template <bool GATHER, int LANES, bool SHORT> __device__ __forceinline__ void materialize_vec_block(const MatVecParams &p, float *__restrict__ cs, unsigned block)
 {
-    __shared__ __align__(16) float cs[COEF_CHUNK];
-    const int64_t n = ((int64_t)blockIdx.x * NT + threadIdx.x) / LANES;
+    const int64_t n = ((int64_t)block * NT + threadIdx.x) / LANES;
     const int part = threadIdx.x % LANES;
     const bool live = n < p.Nw;
     uint32_t a = (uint32_t)n;
@@ -141,6 +141,18 @@ template <bool GATHER, int LANES, bool SHORT> __global__ __launch_bounds__(NT) v
         if (p.scale_bias) acc += load_as_f32(p.scale_bias, p.coef_dtype, 0) * noise1d(a, p.seed);
         p.out[n] = acc;
     }
+}
+template <bool GATHER, int LANES, bool SHORT> __global__ __launch_bounds__(NT) void materialize_vec_kernel(MatVecParams p)
+{
+    __shared__ __align__(16) float cs[COEF_CHUNK];
+    materialize_vec_block<GATHER, LANES, SHORT>(p, cs, blockIdx.x);
+}
+// A weight and its bias, contiguous both: the bias's blocks (16 lanes an element) first.
+template <int LANES, bool SHORT> __global__ __launch_bounds__(NT) void materialize_vec_pair_kernel(MatVecParams weight, MatVecParams bias, unsigned bias_blocks)
+{
+    __shared__ __align__(16) float cs[COEF_CHUNK];
+    if (blockIdx.x < bias_blocks) materialize_vec_block<false, 16, false>(bias, cs, blockIdx.x);
+    else materialize_vec_block<false, LANES, SHORT>(weight, cs, blockIdx.x - bias_blocks);
 }
 
 // Matrix-coef materialise, arbitrary view: one thread per output element (no sharing of noise between rows).
@@ -502,12 +514,13 @@ static void split_plan(int64_t Nw, int64_t k, int64_t *splits, int64_t *span)
     *splits = (cdiv(Nw, sp) > 0 ? cdiv(Nw, sp) : 1) * grad_rows(k);
 }
 
+// lanes per element of a tensor of n values by k terms: as many as fill the chip's 8192 wave slots, of 1, 4, 16
+static int mat_lanes(int64_t n, int64_t k) { return k < 8 ? 1 : n <= (1 << 15) ? 16 : n <= (1 << 17) ? 4 : 1; }
 static int launch_materialize_vec(float *out, const void *coef, int coef_dtype, int64_t k, int64_t Nw, int64_t Q, int64_t sP, int64_t sQ, uint32_t seed,
                                   const void *scale_bias, const int64_t *idx, hipStream_t s)
 {
     const MatVecParams p = {out, coef, scale_bias, idx, k, Nw, Q, sP, sQ, coef_dtype, Nw < (1ll << 32) && Q < (1ll << 32), sQ == 1 && (sP == Q || Nw == Q), seed};
-    // lanes per element: as many as fill the chip's 8192 wave slots, of 1, 4, 16
-    const int lanes = k < 8 ? 1 : Nw <= (1 << 15) ? 16 : Nw <= (1 << 17) ? 4 : 1;
+    const int lanes = mat_lanes(Nw, k);
     const unsigned blocks = (unsigned)cdiv(Nw * lanes, NT);
     auto launch = [&](auto lanes_) {
         constexpr int L = decltype(lanes_)::value;
@@ -608,6 +621,38 @@ extern "C" int rdb_materialize_fwd(float *out, const void *coef, int coef_dtype,
     materialize_mat_generic_kernel<<<(unsigned)cdiv(Nw, NT), NT, 0, s>>>(out, coef, coef_dtype, k, row_len, Nw, Q, sP, sQ, seed,
                                                                          scale_bias);
     return check_launch("materialize_mat_generic_kernel");
+}
+
+extern "C" int rdb_materialize_weight_and_bias(float *weight, int64_t n, const float *coef, int64_t k, uint32_t seed, const float *scale, const rdb_pseudo_bias *bias,
+                                               int64_t bias_n, void *stream)
+{
+    const char *who = "rdb_materialize_weight_and_bias";
+    if (!bias) return set_error(RDB_E_NULL, "%s: bias is NULL", who);
+    if (n < 0 || k < 0 || bias_n < 0 || bias->k < 0 || n > ((int64_t)1 << 38) || bias_n > ((int64_t)1 << 38))
+        return set_error(RDB_E_SHAPE, "%s: n=%lld k=%lld, bias n=%lld k=%lld", who, (long long)n, (long long)k, (long long)bias_n, (long long)bias->k);
+    if ((n > 0 && (!weight || (!coef && k > 0))) || (bias_n > 0 && (!bias->values || (!bias->coef && bias->k > 0)))) return set_error(RDB_E_NULL, "%s: an output or its coefficients are NULL", who);
+    hipStream_t s = (hipStream_t)stream;
+    // Side by side where both are short; a long one's kernel stays as it is, and so do biases that get another number of lanes.
+    if (n > 0 && bias_n > 0 && n * std::max<int64_t>(k, 1) <= MAT_PAIR_HASHES && mat_lanes(bias_n, bias->k) == 16) {
+        const auto params = [](float *out, const float *c, const float *sc, int64_t terms, int64_t len, uint32_t sd) {
+            return MatVecParams{out, c, sc, nullptr, terms, len, len, 0, 1, RDB_F32, len < (1ll << 32), 1, sd};
+        };
+        const MatVecParams w = params(weight, coef, scale, k, n, seed), b = params(bias->values, bias->coef, bias->scale, bias->k, bias_n, bias->seed);
+        const int lanes = mat_lanes(n, k);
+        const unsigned bias_blocks = (unsigned)cdiv(bias_n * 16, NT), blocks = bias_blocks + (unsigned)cdiv(n * lanes, NT);
+        auto launch = [&](auto lanes_) {
+            constexpr int L = decltype(lanes_)::value;
+            if (k <= MAT_SHORT) materialize_vec_pair_kernel<L, true><<<blocks, NT, 0, s>>>(w, b, bias_blocks);
+            else materialize_vec_pair_kernel<L, false><<<blocks, NT, 0, s>>>(w, b, bias_blocks);
+        };
+        if (lanes == 16) launch(std::integral_constant<int, 16>{});
+        else if (lanes == 4) launch(std::integral_constant<int, 4>{});
+        else launch(std::integral_constant<int, 1>{});
+        return check_launch("materialize_vec_pair_kernel");
+    }
+    if (n > 0)
+        if (int rc = launch_materialize_vec(weight, coef, RDB_F32, k, n, n, 0, 1, seed, scale, nullptr, s)) return rc;
+    return bias_n > 0 ? launch_materialize_vec(bias->values, bias->coef, RDB_F32, bias->k, bias_n, bias_n, 0, 1, bias->seed, bias->scale, nullptr, s) : RDB_OK;
 }
 
 extern "C" int64_t rdb_materialize_bwd_workspace_bytes(int64_t coef_rows, int64_t k, int64_t row_len, int64_t Nw)

@@ -216,6 +216,17 @@ struct Bias {
         if (!coef) return Tensor();
         return (seed < 0 ? *coef : coef_values(*coef, scale, n, seed)).to(dtype).contiguous();
     }
+    // ... as the library's calls take it that form them into `values` on the side (see beside); the tensors are the caller's
+    rdb_pseudo_bias ref(const Tensor &c, const Tensor &s, const Tensor &values) const
+    {
+        return {c.data_ptr<float>(), s.defined() ? s.data_ptr<float>() : nullptr, values.data_ptr<float>(), c.numel(), (uint32_t)seed};
+    }
+    // Whether the values may be formed by a launch that a layer with fp32 rows makes anyway; the bounds: the summation order of coef_values
+    bool beside(int64_t n, at::ScalarType dtype) const
+    {
+        return coef && seed >= 0 && dtype == at::kFloat && coef->scalar_type() == at::kFloat && coef->numel() >= 8 && n > 0 && n <= (1 << 15) &&
+               (!scale || !scale->defined() || (scale->scalar_type() == at::kFloat && scale->numel() >= 1));
+    }
     // what its gradient needs of it: whether there is one, length, seed, dtypes
     std::vector<int64_t> meta() const
     {
@@ -369,11 +380,19 @@ class OneCallLinear : public Function<OneCallLinear> {
             return linear_fwd(x0, coefs, l, scale_bias, b);
         }
         const c10::OptionalDeviceGuard guard(x.device());
-        const Tensor c = coefs.contiguous(), sb = scale_bias ? scale_bias->to(c.scalar_type()) : Tensor(), bv = b.values(l.out_f, x.scalar_type());
+        const Tensor c = coefs.contiguous(), sb = scale_bias ? scale_bias->to(c.scalar_type()) : Tensor();
         const Tensor xn = near_act(x);
         Tensor y = at::empty({x.size(0), l.out_f}, x.options()), kept = bytes(keep, x);
-        check(rdb_linear_fwd_kept(y.data_ptr(), l.out_f, kept.data_ptr(), xn.data_ptr(), xn.stride(0), c.data_ptr(), ptr(sb), ptr(bv), &d, stream_of(x)),
-              "rdb_linear_fwd_kept");
+        if (b.beside(l.out_f, x.scalar_type())) {
+            const Tensor bc = b.coef->contiguous(), bs = b.scale && b.scale->defined() ? b.scale->contiguous() : Tensor(), bv = at::empty({l.out_f}, x.options());
+            const rdb_pseudo_bias pb = b.ref(bc, bs, bv);
+            check(rdb_linear_fwd_kept_pseudo_bias(y.data_ptr(), l.out_f, kept.data_ptr(), xn.data_ptr(), xn.stride(0), c.data_ptr(), ptr(sb), &pb, &d, stream_of(x)),
+                  "rdb_linear_fwd_kept");
+        } else {
+            const Tensor bv = b.values(l.out_f, x.scalar_type());
+            check(rdb_linear_fwd_kept(y.data_ptr(), l.out_f, kept.data_ptr(), xn.data_ptr(), xn.stride(0), c.data_ptr(), ptr(sb), ptr(bv), &d, stream_of(x)),
+                  "rdb_linear_fwd_kept");
+        }
         ctx->save_for_backward({scale_bias ? x0 : Tensor(), coefs, scale_bias.value_or(Tensor()), kept});
         return y;
     }
@@ -633,8 +652,21 @@ class VectorLinear : public Function<VectorLinear> {
     {
         const Bias b{bias, bias_scale, bias_seed};
         const c10::OptionalDeviceGuard guard(x0.device());
-        const Tensor W = coef_values(coef, scale, l.out_f * l.in_f, l.seed).view({l.out_f, l.in_f});
-        Tensor y = values(x0, W, b, l);
+        Tensor W, bv;
+        if (b.beside(l.out_f, x0.scalar_type()) && coef.scalar_type() == at::kFloat && (!scale || !scale->defined() || scale->scalar_type() == at::kFloat)) {
+            const Tensor c = coef.contiguous(), sc = scale && scale->defined() ? scale->contiguous() : Tensor();
+            const Tensor bc = b.coef->contiguous(), bs = b.scale && b.scale->defined() ? b.scale->contiguous() : Tensor();
+            W = at::empty({l.out_f, l.in_f}, c.options());
+            bv = at::empty({l.out_f}, c.options());
+            const rdb_pseudo_bias pb = b.ref(bc, bs, bv);
+            check(rdb_materialize_weight_and_bias(W.data_ptr<float>(), W.numel(), c.data_ptr<float>(), c.numel(), l.seed, sc.defined() ? sc.data_ptr<float>() : nullptr,
+                                                  &pb, l.out_f, stream_of(c)),
+                  "rdb_materialize_weight_and_bias");
+        } else {
+            W = coef_values(coef, scale, l.out_f * l.in_f, l.seed).view({l.out_f, l.in_f});
+            bv = b.values(l.out_f, x0.scalar_type());
+        }
+        Tensor y = values(x0, W, bv, l);
         const bool keep = ctx != nullptr && W.numel() <= x0.numel() + y.numel();
         if (ctx) {
             ctx->save_for_backward({x0, coef, scale.value_or(Tensor()), keep && x0.requires_grad() ? W : Tensor()});
@@ -644,11 +676,11 @@ class VectorLinear : public Function<VectorLinear> {
         }
         return y;
     }
-    static Tensor values(const Tensor &x0, const Tensor &W, const Bias &b, const Layer &l)
+    static Tensor values(const Tensor &x0, const Tensor &W, const Tensor &bias, const Layer &l)
     {
         auto sizes = x0.sizes().vec();
         sizes.back() = l.out_f;
-        return product(at::empty(sizes, x0.options()), act(x0.reshape({-1, l.in_f})), false, W, false, b.values(l.out_f, x0.scalar_type()));
+        return product(at::empty(sizes, x0.options()), act(x0.reshape({-1, l.in_f})), false, W, false, bias);
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {

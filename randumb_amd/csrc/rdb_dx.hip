@@ -508,15 +508,17 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             const int items = make_tns_params(bs.tn, dx, lddx, workspace, d, num_cus);
             bs.red = red;
             bs.tn_blocks = xcd_grid_size(items);
-            int rblocks = (int)cdiv(red.n / 4 * red.splits, ST_THREADS * 16);   // about 16 loads of 16 bytes a thread
-            if (rblocks > num_cus / 2) rblocks = num_cus / 2;
-            // a block of this kernel has a compute unit to itself: where the product's blocks leave units free, no more reduction
+            // One element (of all splits) a thread while there are units for it: a turn is a round trip to memory of 1.5 us, and with 16 loads
+            // a thread a few blocks were still adding when the product was done (528 tokens x 384 -> 1536, k = 112: 16 blocks 7.6 us, 84
+            // blocks 3.6; 3008 x 768 -> 2304, k = 96: 5.7 -> 4.1).
+            int rblocks = (int)std::min<int64_t>(cdiv(red.n / 4, ST_THREADS), num_cus);
+            // A block of this kernel has a compute unit to itself: where the product's blocks leave units free, no more reduction
             // blocks than those, so that the launch is one round of blocks (8192 tokens x 768 -> 3072, k = 256, 64 units: 9.8 us against
-            // 11.2 with 128 blocks).  Less than half of the blocks would still be adding long after the product is done, and a second
+            // 11.2 with 128 blocks).  Less than a quarter of the chip would still be adding long after the product is done, and a second
             // round is cheaper: 6784 x 576 -> 1728, k = 256, 8 units: 11.6 against 50.4; 4000 x 960 -> 4096, k = 128, 32 units: 8.6
             // against 20.0; 8192 x 448 -> 4096, k = 256, 32 units: 11.6 against 18.4.
             const int spare = num_cus - bs.tn_blocks;
-            if (spare > 0 && rblocks > spare && rblocks <= 2 * spare) rblocks = spare;
+            if (spare > 0 && rblocks > spare && std::min(rblocks, num_cus / 2) <= 2 * spare) rblocks = spare;
             if (rblocks < 1) rblocks = 1;
             if (direct) rblocks = 0;
             return with_stationary_variant(bs.tn, [&](auto kg, auto aux) {
@@ -536,7 +538,7 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
         const int tn_items = make_tn_params(b.tn, dx, lddx, workspace, d);
         b.tn_blocks = xcd_grid_size(tn_items);
         b.red = red;
-        int red_blocks = (int)cdiv(b.red.n / 4 * b.red.splits, 256 * 16);
+        int red_blocks = (int)cdiv(b.red.n / 4 * b.red.splits, 256 * 16);   // two blocks a unit: no gain from more
         if (red_blocks > num_cus) red_blocks = num_cus;
         if (red_blocks < 1) red_blocks = 1;
         if (direct) red_blocks = 0;

@@ -6,8 +6,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# units left free of 256, with 256 tokens and 64 features a unit of work: 8 (9 x 27 blocks, in groups of 8), 64 (6 x 32), 32 (7 x 32), none (8 x 32)
-@pytest.mark.parametrize("T,in_f,out_f,k", [(6784, 576, 264, 168), (8192, 384, 1160, 256), (8192, 448, 1160, 256), (8000, 512, 520, 72)])
+# units left free of 256, with 256 tokens and 64 features a unit of work: 8 (9 x 27 blocks, in groups of 8), 64 (6 x 32), 32 (7 x 32), none (8 x 32),
+# more than elements to add (one block, and a part of a second)
+@pytest.mark.parametrize("T,in_f,out_f,k", [(6784, 576, 264, 168), (8192, 384, 1160, 256), (8192, 448, 1160, 256), (8000, 512, 520, 72), (528, 64, 32, 64), (528, 384, 40, 64)])
 def test_coefficient_gradient_against_float64(T, in_f, out_f, k):
     from randumb_amd import hip
 

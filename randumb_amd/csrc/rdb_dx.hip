@@ -24,7 +24,7 @@ constexpr int X_BK = 64;
 // small (tokens x k), so the token tile is kept short to have a block for every compute unit; loads run two stages ahead.
 constexpr int K1_BC = 128, K1_BT = 64;
 // pipeline shape of the dy.C blocks that take C^T straight into registers: contraction per stage, stages per unrolled trip,
-// how many stages ahead dy is loaded, depth of the fragment ring in stages, wave priority
+// how many stages ahead dy is loaded, wave priority
 #ifndef RDB_DYC_BKD
 #define RDB_DYC_BKD 128
 #endif
@@ -33,9 +33,6 @@ constexpr int K1_BC = 128, K1_BT = 64;
 #endif
 #ifndef RDB_DYC_DSTG
 #define RDB_DYC_DSTG 2
-#endif
-#ifndef RDB_DYC_RD
-#define RDB_DYC_RD 1
 #endif
 #ifndef RDB_DYC_PRIO
 #define RDB_DYC_PRIO 2
@@ -125,8 +122,9 @@ __device__ __forceinline__ void dyc_block(const DyCParams &p, bf16_t *lds, int b
 }
 
 // The same block with C taken from its transposed, fragment-ordered copy: only dy passes through LDS.  The four waves split
-// the coefficient rows (one 32-row block each, no fragment loaded twice) and share the 64 tokens.
-__device__ __forceinline__ void dyc_block_direct(const DyCParams &p, bf16_t *lds, int block)
+// the coefficient rows (one 32-row block each, no fragment loaded twice) and share the 64 tokens.  RD: how many stages ahead C's fragments are
+// loaded (bwd_dc_dyc_kernel).
+template <int RD> __device__ __forceinline__ void dyc_block_direct(const DyCParams &p, bf16_t *lds, int block)
 {
     const int tiles = p.tiles_c * p.tiles_t, items = p.part ? tiles * p.ranges : tiles, wr = xcd_work_item(block, items);
     if (wr >= items) return;
@@ -145,7 +143,7 @@ __device__ __forceinline__ void dyc_block_direct(const DyCParams &p, bf16_t *lds
 #pragma unroll
         for (int ni = 0; ni < K1_BT / 32; ++ni) acc[0][ni] = zero16();
         GlobalOperand<K1_BT, BKD, K_CONT> opdy = {p.dy, p.lddy, tok0, p.tokens, o_end, (int64_t)(p.tokens - 1) * p.lddy + p.out_f};
-        direct_mainloop<K1_BT / 32, 1, BKD / 16, false, RDB_DYC_TRIP, RDB_DYC_DSTG, RDB_DYC_RD>(acc, lds, opdy, fc, o_begin, (o_end - o_begin + BKD - 1) / BKD, 0,
+        direct_mainloop<K1_BT / 32, 1, BKD / 16, false, RDB_DYC_TRIP, RDB_DYC_DSTG, RD>(acc, lds, opdy, fc, o_begin, (o_end - o_begin + BKD - 1) / BKD, 0,
                                                                                                lane);
         if (last == range) break;
         __syncthreads();   // the next range begins by writing the stage buffers
@@ -251,7 +249,11 @@ struct BwdAParams {
     int dc_blocks;  // multiple of 8, so both parts keep their die assignment
 };
 
-__global__ __launch_bounds__(256, 2) void bwd_dc_dyc_kernel(BwdAParams p)
+// RD: see dyc_block_direct.  Where the blocks of t = dy . C take half the compute units or fewer, each is a chain of stages that wait for C's
+// fragments, and two stages ahead shorten it (528 tokens x 384 -> 1536, k = 112, 9 blocks of 12 stages: 14.2 us -> 11.7; 700 x 2000 -> 1000, k = 128:
+// 10.0 -> 8.6; 5000 x 1000 -> 1000, k = 64: 10.6 -> 9.4); with a block or more a unit the others' work fills the waits, and the 24 registers are missed
+// (8192 x 768 -> 3072, k = 256: 34.5 -> 36.5; 4096 tokens: 27.7 -> 28.2).
+template <int RD> __global__ __launch_bounds__(256, 2) void bwd_dc_dyc_kernel(BwdAParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
@@ -259,7 +261,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dc_dyc_kernel(BwdAParams p)
         dc_block_direct(p.dc, lds, blockIdx.x);
     } else {
         if (p.dyc.ctf && *p.dyc.ctf_flag)   // the forward pass left the transposed coefficients in the state
-            dyc_block_direct(p.dyc, lds, blockIdx.x - p.dc_blocks);
+            dyc_block_direct<RD>(p.dyc, lds, blockIdx.x - p.dc_blocks);
         else
             dyc_block(p.dyc, lds, blockIdx.x - p.dc_blocks);
     }
@@ -337,15 +339,16 @@ int64_t linear_bwd_projected_workspace(const rdb_linear_desc *d, int num_cus, bo
 // Ranges of t = dy . C where its tiles are half the compute units or fewer and each contracts 2048 output features or more: a block walks
 // through them at 1 us a stage of 128 while the launch's other blocks are long done (1178 tokens x 640 -> 6520, k = 160: 38 blocks of 51
 // stages; the whole backward pass 57 -> 30 us with the launch that adds the ranges up; 2048 x 4096 -> 11008, k = 256: 91 -> 61; at the
-// line, 300 x 512 -> 2048, k = 64: 21.7 -> 20.0, 2048 x 1024 -> 2048, k = 96: 19.1 -> 18.5).  At least 1024 output features a range, at
-// most eight ranges.  k <= 256 only: the 256-wide tiles, which take longer ones where there are enough of them, contract in one range,
+// line, 300 x 512 -> 2048, k = 64: 21.7 -> 20.0, 2048 x 1024 -> 2048, k = 96: 19.1 -> 18.5).  At least 512 output features a range, four stages
+// (with 1024, the two launches of 300 x 512 -> 2048, k = 64: 14.5 us, now 11.1; 1056 x 768 -> 3072, k = 240: 19.6, now 17.4; 384 gains nothing
+// more), at most eight ranges.  k <= 256 only: the 256-wide tiles, which take longer ones where there are enough of them, contract in one range,
 // and both give the same bits.  The rule knows nothing of workspaces: without room for the ranges' sums a block adds its tile's
 // ranges up itself, to the same bits.
 static int dyc_ranges(const rdb_linear_desc *d, int num_cus, int *range_len)
 {
     const int64_t tiles = cdiv(d->k, K1_BC) * cdiv(d->tokens, K1_BT);
-    int64_t r = std::min<int64_t>(std::min<int64_t>(num_cus / tiles, d->out_f / 1024), 8);
-    if (r < 2 || d->k > ST_KMAX) r = 1;
+    int64_t r = std::min<int64_t>(std::min<int64_t>(num_cus / tiles, d->out_f / 512), 8);
+    if (r < 2 || d->out_f < 2048 || d->k > ST_KMAX) r = 1;
     *range_len = (int)(cdiv(cdiv(d->out_f, r), 128) * 128);
     return (int)cdiv(d->out_f, *range_len);
 }
@@ -485,8 +488,10 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             rc = linear_bwd_big(workspace, a.dc.partial, direct && dc_bf16, dy, lddy, z, coef, d, num_cus, true, true, s);
         } else {
             size_t smem = smem_dc > smem_dyc ? smem_dc : smem_dyc;
-            if (int rl = reserve_lds(reinterpret_cast<const void *>(bwd_dc_dyc_kernel), smem, "bwd_dc_dyc_kernel")) return rl;
-            bwd_dc_dyc_kernel<<<a.dc_blocks + xcd_grid_size(p1.tiles_c * p1.tiles_t * (a.dyc.part ? a.dyc.ranges : 1)), 256, smem, s>>>(a);
+            const int dyc_items = p1.tiles_c * p1.tiles_t * (a.dyc.part ? a.dyc.ranges : 1);
+            auto kernel = dyc_items * 2 <= num_cus ? bwd_dc_dyc_kernel<2> : bwd_dc_dyc_kernel<1>;
+            if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem, "bwd_dc_dyc_kernel")) return rl;
+            kernel<<<a.dc_blocks + xcd_grid_size(dyc_items), 256, smem, s>>>(a);
             rc = check_launch("bwd_dc_dyc_kernel");
             if (!rc && a.dyc.part) {
                 const int k8 = a.dyc.frag_ksteps * 2, pieces = (int)(cdiv(d->tokens, 32) * 32) * k8;

@@ -221,6 +221,7 @@ inline int make_dc_params(DcParams &p, float *dcoef, const void *dy, int64_t ldd
 // forward product / first backward launch, and the launches.  `dc`: where the coefficient gradient's sums are stored.
 bool big_fwd_applies(const rdb_linear_desc *d, int num_cus);
 bool big_bwd_applies(const rdb_linear_desc *d, int num_cus);
+bool big_bwd_enough(const rdb_linear_desc *d, int num_cus);
 int linear_fwd_big(void *y, int64_t ldy, const void *state, const void *coef, const void *bias, const rdb_linear_desc *d, int num_cus, hipStream_t s);
 int linear_bwd_big(void *t, void *dc, bool dc_bf16, const void *dy, int64_t lddy, const void *state, const void *coef, const rdb_linear_desc *d,
                    int num_cus, bool want_t, bool want_dc, hipStream_t s);

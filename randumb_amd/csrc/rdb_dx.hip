@@ -164,7 +164,7 @@ template <int RD> __device__ __forceinline__ void dyc_block_direct(const DyCPara
     RDB_STAMP(3);
 }
 
-// t from the ranges' sums, added in range order: eight coefficients of a token a thread, in fragment order (as store_tile_bf16_frag
+// t from the ranges' sums, added in range order: eight coefficients of a token a thread, row-major or in fragment order (as store_tile_bf16_frag
 // writes it: tokens padded to 32 and coefficients to a multiple of 64 with zeros, times 2^-31)
 __global__ __launch_bounds__(256) void dyc_sum_kernel(DyCParams p, int pieces, int k8)
 {
@@ -191,9 +191,12 @@ __global__ __launch_bounds__(256) void dyc_sum_kernel(DyCParams p, int pieces, i
                 hi += b[i];
             }
     }
-    lo *= 4.656612873077392578125e-10f;
-    hi *= 4.656612873077392578125e-10f;
-    bf16_t *dst = p.t + ((int64_t)(tok >> 5) * p.frag_ksteps + (m >> 4)) * 512 + (((m >> 3) & 1) * 32 + (tok & 31)) * 8;
+    bf16_t *dst = p.t + (int64_t)tok * p.k + m;
+    if (p.frag_ksteps) {
+        lo *= 4.656612873077392578125e-10f;
+        hi *= 4.656612873077392578125e-10f;
+        dst = p.t + ((int64_t)(tok >> 5) * p.frag_ksteps + (m >> 4)) * 512 + (((m >> 3) & 1) * 32 + (tok & 31)) * 8;
+    }
     const i32x4 h = {(int)f32x2_to_bf16x2(lo[0], lo[1]), (int)f32x2_to_bf16x2(lo[2], lo[3]), (int)f32x2_to_bf16x2(hi[0], hi[1]),
                      (int)f32x2_to_bf16x2(hi[2], hi[3])};
     *reinterpret_cast<i32x4 *>(dst) = h;
@@ -336,19 +339,20 @@ int64_t linear_bwd_projected_workspace(const rdb_linear_desc *d, int num_cus, bo
     return align256(linear_dx_factored_workspace(d)) + (int64_t)dc.splits * d->out_f * d->k * (int64_t)sizeof(float);
 }
 
-// Ranges of t = dy . C where its tiles are half the compute units or fewer and each contracts 2048 output features or more: a block walks
-// through them at 1 us a stage of 128 while the launch's other blocks are long done (1178 tokens x 640 -> 6520, k = 160: 38 blocks of 51
-// stages; the whole backward pass 57 -> 30 us with the launch that adds the ranges up; 2048 x 4096 -> 11008, k = 256: 91 -> 61; at the
-// line, 300 x 512 -> 2048, k = 64: 21.7 -> 20.0, 2048 x 1024 -> 2048, k = 96: 19.1 -> 18.5).  At least 512 output features a range, four stages
-// (with 1024, the two launches of 300 x 512 -> 2048, k = 64: 14.5 us, now 11.1; 1056 x 768 -> 3072, k = 240: 19.6, now 17.4; 384 gains nothing
-// more), at most eight ranges.  k <= 256 only: the 256-wide tiles, which take longer ones where there are enough of them, contract in one range,
-// and both give the same bits.  The rule knows nothing of workspaces: without room for the ranges' sums a block adds its tile's
-// ranges up itself, to the same bits.
+// Ranges of t = dy . C where its tiles are half the compute units or fewer and each contracts 2048 output features or more (k > 256: 2560): a
+// block walks through them at 0.75 to 1 us a stage of 128 while the launch's other blocks are long done (the two launches, and the one without:
+// 300 tokens x 512 -> 2560, k = 64: 11.1 us, 13.7; 2000, k = 256: 19.4, 20.3; 300 x 512 -> 3584, k = 512: 15.9, 27.7; at 2048 features, k = 64, 200
+// and 256: 10.9, 11.4; 14.2, 13.0; 17.5, 19.7; with k = 304 16.6, 14.1).  At least 512 output features a range, four stages (with 1024: 446 x 792 -> 4168, k = 64: 16.4 us, now 12.1; 1056 x 768 -> 3072, k =
+// 240: 19.0, now 16.7; 384 gains nothing more), at most eight ranges.  Up to five eighths of the units and from 4096 features on, two ranges still
+// pay (3010 x 1024 -> 7736, k = 272, 144 tiles: 68 -> 54 us; 158 tiles: 76 either way; 192: 59 -> 69, and 142 tiles of 3072 features 30 -> 36).
+// Not where the 256-wide tiles take the layer when they are switched on: those contract in one range, and both give the same bits.  The rule
+// knows nothing of workspaces: without room for the ranges' sums a block adds its tile's ranges up itself, to the same bits.
 static int dyc_ranges(const rdb_linear_desc *d, int num_cus, int *range_len)
 {
     const int64_t tiles = cdiv(d->k, K1_BC) * cdiv(d->tokens, K1_BT);
     int64_t r = std::min<int64_t>(std::min<int64_t>(num_cus / tiles, d->out_f / 512), 8);
-    if (r < 2 || d->out_f < 2048 || d->k > ST_KMAX) r = 1;
+    if (r < 2 && tiles * 8 <= num_cus * 5 && d->out_f >= 4096) r = 2;
+    if (r < 2 || d->out_f < (d->k <= ST_KMAX ? 2048 : 2560) || big_bwd_enough(d, num_cus)) r = 1;
     *range_len = (int)(cdiv(cdiv(d->out_f, r), 128) * 128);
     return (int)cdiv(d->out_f, *range_len);
 }
@@ -461,7 +465,7 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
         dc_params_from_state(a.dc, z, d);
         // one token range only (the 256-wide tiles always have one): its sums are the result, stored straight into dcoef, and
         // nothing is left to add up
-        const bool big = big_bwd_applies(d, num_cus) && !tn_stationary_ok(d, lddx);
+        const bool big = big_bwd_applies(d, num_cus) && !tn_stationary_ok(d, lddx) && p1.ranges == 1;   // more than one: only when they are forced on
         const bool direct = !accumulate && (big || (a.dc.splits == 1 && !dc_bf16));
         a.dc.partial = direct ? dcoef : reinterpret_cast<float *>(static_cast<char *>(workspace) + align256(linear_dx_factored_workspace(d)));
         a.dyc = p1;
@@ -474,10 +478,8 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
         }
         if (tn_stationary_ok(d, lddx)) a.dyc.frag_ksteps = (int)cdiv(d->k, 64) * 4;   // the t.N kernel below keeps t in registers
         const int64_t base = align256(linear_bwd_projected_workspace(d, num_cus, accumulate || dc_bf16));
-        if (a.dyc.frag_ksteps) {
-            if (a.dyc.ranges > 1 && workspace_bytes >= base + align256(a.dyc.ranges * d->tokens * d->k * (int64_t)sizeof(float)))
-                a.dyc.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + base);
-        }
+        if (a.dyc.ranges > 1 && workspace_bytes >= base + align256(a.dyc.ranges * d->tokens * d->k * (int64_t)sizeof(float)))
+            a.dyc.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + base);
         a.dc_blocks = xcd_grid_size(dc_items);
         int rc = RDB_OK;
         const int red_splits = big ? 1 : a.dc.splits;
@@ -494,7 +496,8 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             kernel<<<a.dc_blocks + xcd_grid_size(dyc_items), 256, smem, s>>>(a);
             rc = check_launch("bwd_dc_dyc_kernel");
             if (!rc && a.dyc.part) {
-                const int k8 = a.dyc.frag_ksteps * 2, pieces = (int)(cdiv(d->tokens, 32) * 32) * k8;
+                const int k8 = a.dyc.frag_ksteps ? a.dyc.frag_ksteps * 2 : (int)d->k / 8;
+                const int pieces = (int)(a.dyc.frag_ksteps ? cdiv(d->tokens, 32) * 32 : d->tokens) * k8;
                 dyc_sum_kernel<<<(unsigned)cdiv(pieces, 256), 256, 0, s>>>(a.dyc, pieces, k8);
                 rc = check_launch("dyc_sum_kernel");
             }

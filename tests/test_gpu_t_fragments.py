@@ -1,5 +1,5 @@
-"""t = dy . C with C's fragments loaded one or two stages of 128 output features ahead, by how many blocks there are, and in ranges of 512
-output features or more."""
+"""t = dy . C with C's fragments loaded one or two stages of 128 output features ahead, by how many blocks there are, and from 2048 output
+features on in ranges of 512 or more."""
 import pytest
 import torch
 
@@ -16,9 +16,10 @@ def _backward(T, in_f, out_f, k, n):
     return x, dy, c, hip.linear_bwd_projected(dy, hip.linear_project(x, k, out_f, 9, c), c, in_f, 9)
 
 
-# one stage, two, three (the last of them past the end), a part of the last; 2048 features and more: two ranges to eight, the last one short
+# one stage, two, three (the last of them past the end), a part of the last; 2048 features and more: four ranges, two to eight, the last one short
 @pytest.mark.parametrize("T,in_f,out_f,k", [(1, 64, 8, 8), (65, 96, 136, 40), (200, 64, 384, 136), (130, 72, 1000, 256), (300, 64, 2048, 64),
-                                            (1056, 72, 3080, 240), (97, 64, 8200, 24), (2050, 64, 2056, 200)])
+                                            (1056, 72, 3080, 240), (97, 64, 8200, 24), (2050, 64, 2056, 200),
+                                            (97, 64, 2568, 264), (300, 520, 8192, 512), (2800, 320, 4104, 304)])
 def test_against_float64(T, in_f, out_f, k):
     from randumb_amd import hip
 

@@ -438,7 +438,7 @@ struct BigRBiasParams {
     bf16_t *dst;            // [tokens x cols]
     const bf16_t *scale;    // one value
     const bf16_t *other;    // DOT: [tokens x cols], what the product without s is reduced against: one sum a tile, in tile order
-    float *dot_part;
+    BlockSum dscale;
     int64_t ld_src, ld_dst, ld_other;
     int tokens, cols, contraction, tiles_a, tiles_t;
 };
@@ -468,8 +468,12 @@ template <bool DOT> __global__ __launch_bounds__(256, 1) void big_rbias_kernel(B
         pb = PB{p.src, p.ld_src, (w / p.tiles_a) * BR_TOK, p.tokens, p.contraction, (int64_t)(p.tokens - 1) * p.ld_src + p.contraction};
         big_prefetch(regs, pa, pb, 0);
     };
+    auto add_up = [&]() { sum_shares(p.dscale, total, 1, 0, nblk, reinterpret_cast<float *>(lds)); };
     int w = next();
-    if (w < 0) return;
+    if (w < 0) {   // the grid is rounded up to a multiple of 8: blocks without a tile are counted too
+        if (DOT) add_up();
+        return;
+    }
     request(w);
     const float sval = bf16_to_f32(*p.scale);
     const __amdgpu_buffer_rsrc_t rs_d = __builtin_amdgcn_make_buffer_rsrc(p.dst, 0, (int)(((int64_t)(p.tokens - 1) * p.ld_dst + p.cols) * 2), 0x00020000);
@@ -547,12 +551,13 @@ template <bool DOT> __global__ __launch_bounds__(256, 1) void big_rbias_kernel(B
             for (int o = 32; o >= 1; o >>= 1) dot += __shfl_xor(dot, o, 64);
             if (lane == 0) wsum[wave] = dot;
             __syncthreads();
-            if (t == 0) p.dot_part[w] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+            if (t == 0) leave_share(p.dscale, w, (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]));
             __syncthreads();
         }
         if (wn < 0) break;
         w = wn;
     }
+    if (DOT) add_up();
 }
 
 // ----------------------------------------------------------------------------------------------- y = z . C^T + s * x . R^T (+ bias)
@@ -697,9 +702,10 @@ int linear_fwd_big(void *y, int64_t ldy, const void *state, const void *coef, co
 // 2^-31: a product with either has the same bits.  Fragment order, because a stage of 64 columns then is consecutive kilobytes, not 128
 // bytes of each of 256 rows (4096 tokens x 4096, k = 1024, rows of 8 KB: z 66 -> 62 us; dx, rows of 2 KB: the same).
 __global__ __launch_bounds__(256) void noise_frag_bf16_kernel(bf16_t *__restrict__ out, uint32_t pieces, uint32_t ksteps, uint32_t rows, uint32_t cols,
-                                                              uint32_t row_step, uint32_t col_step, uint32_t seed)
+                                                              uint32_t row_step, uint32_t col_step, uint32_t seed, unsigned int *cleared)
 {
     const uint32_t e = blockIdx.x * 256u + threadIdx.x;
+    if (e == 0 && cleared) *cleared = 0u;   // a word that a later launch counts in
     if (e >= pieces) return;
     const uint32_t lane = e & 63u, unit = e >> 6, rb = unit / ksteps, ks = unit - rb * ksteps, r = rb * 32u + (lane & 31u), c = ks * 16u + (lane >> 5) * 8u;
     i32x4 h = {0, 0, 0, 0};
@@ -715,11 +721,12 @@ __global__ __launch_bounds__(256) void noise_frag_bf16_kernel(bf16_t *__restrict
 }
 // rows rounded up to 32, columns to 64
 static int64_t noise_frag_bytes(int64_t rows, int64_t cols) { return cdiv(rows, 32) * 32 * cdiv(cols, 64) * 64 * (int64_t)sizeof(bf16_t); }
-static int launch_noise_frag(void *out, int64_t rows, int64_t cols, uint32_t row_step, uint32_t col_step, uint32_t seed, hipStream_t s)
+static int launch_noise_frag(void *out, int64_t rows, int64_t cols, uint32_t row_step, uint32_t col_step, uint32_t seed, hipStream_t s,
+                             unsigned int *cleared = nullptr)
 {
     const uint32_t pieces = (uint32_t)(noise_frag_bytes(rows, cols) / 16);
     noise_frag_bf16_kernel<<<(unsigned)cdiv(pieces, 256), 256, 0, s>>>(static_cast<bf16_t *>(out), pieces, (uint32_t)(cdiv(cols, 64) * 4), (uint32_t)rows,
-                                                                       (uint32_t)cols, row_step, col_step, seed);
+                                                                       (uint32_t)cols, row_step, col_step, seed, cleared);
     return check_launch("noise_frag_bf16_kernel");
 }
 
@@ -804,33 +811,34 @@ int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cu
     return bytes;
 }
 
-// dst[t, a] += s * sum_c src[t, c] * noise1d(a * sR + c * sK); with `other` also one sum per tile to dot_part, *tiles of them.  The caller
-// has checked alignments and extents.
+// dst[t, a] += s * sum_c src[t, c] * noise1d(a * sR + c * sK); with `other` also the sum of the product's elements times its, to dscale, with one
+// share per tile in dot_part and a word behind the table.  The caller has checked alignments and extents.
 int linear_rbias_big(void *dst, int64_t ld_dst, int64_t cols, const void *src, int64_t ld_src, int64_t contraction, uint32_t sR, uint32_t sK,
-                     const void *scale, const rdb_linear_desc *d, void *table, const void *other, int64_t ld_other, float *dot_part, int *tiles,
+                     const void *scale, const rdb_linear_desc *d, void *table, const void *other, int64_t ld_other, float *dot_part, void *dscale, int dscale_dtype,
                      int num_cus, hipStream_t s)
 {
-    if (int rc = launch_noise_frag(table, cols, contraction, sR * SQ5_N1, sK * SQ5_N1, d->seed, s)) return rc;
     BigRBiasParams p;
+    p.tiles_a = (int)cdiv(cols, BG);
+    p.tiles_t = (int)cdiv(d->tokens, BR_TOK);
+    const int tiles = p.tiles_a * p.tiles_t;
+    p.dscale = {dot_part, other ? reinterpret_cast<unsigned int *>(static_cast<char *>(table) + noise_frag_bytes(cols, contraction)) : nullptr, dscale,
+                dscale_dtype == RDB_BF16};
+    if (int rc = launch_noise_frag(table, cols, contraction, sR * SQ5_N1, sK * SQ5_N1, d->seed, s, p.dscale.arrived)) return rc;
     p.noise = static_cast<const bf16_t *>(table);
     p.src = static_cast<const bf16_t *>(src);
     p.dst = static_cast<bf16_t *>(dst);
     p.scale = static_cast<const bf16_t *>(scale);
     p.other = static_cast<const bf16_t *>(other);
-    p.dot_part = dot_part;
     p.ld_src = ld_src;
     p.ld_dst = ld_dst;
     p.ld_other = ld_other;
     p.tokens = (int)d->tokens;
     p.cols = (int)cols;
     p.contraction = (int)contraction;
-    p.tiles_a = (int)cdiv(cols, BG);
-    p.tiles_t = (int)cdiv(d->tokens, BR_TOK);
-    *tiles = p.tiles_a * p.tiles_t;
     constexpr size_t stages = big_smem<BG, BR_TOK, FragTile<BG, 64>, OperandTile<BR_TOK, 64, K_CONT>>();
     static_assert((size_t)4 * 32 * (BG / 2 + 4) * sizeof(float) <= stages, "the epilogue's patches fit the pipeline's LDS");
-    if (other) return launch_big(big_rbias_kernel<true>, p, *tiles, num_cus, stages, s, "big_rbias_kernel<dot>");
-    return launch_big(big_rbias_kernel<false>, p, *tiles, num_cus, stages, s, "big_rbias_kernel");
+    if (other) return launch_big(big_rbias_kernel<true>, p, tiles, num_cus, stages, s, "big_rbias_kernel<dot>");
+    return launch_big(big_rbias_kernel<false>, p, tiles, num_cus, stages, s, "big_rbias_kernel");
 }
 
 // y = z . C^T + s * x . R^T (+ bias) from the state, R in `table` (rbias_big_table_bytes of out_f columns)

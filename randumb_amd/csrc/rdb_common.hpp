@@ -222,6 +222,46 @@ __device__ __forceinline__ void release_tags(unsigned long long *slots, int n, u
     if (old == (unsigned int)(consumers - 1) && lane < n) __hip_atomic_store(slots + lane, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A sum over the blocks of a launch without a launch of its own: every block leaves its share and counts itself, and the last one adds the
+// shares up, in an order that does not depend on who that is.  Counting one word costs 10 ns a block (1248 blocks: 13 us), so the blocks come in
+// groups: the last of a group counts it.
+struct BlockSum {
+    float *part;             // one value per item
+    unsigned int *arrived;   // a word for the groups, then one per group; zero when the launch begins (an earlier launch's business)
+    void *out;
+    int out_bf16;
+};
+// one thread of the block (always the same one)
+__device__ __forceinline__ void leave_share(const BlockSum &q, int item, float v)
+{
+    __hip_atomic_store(q.part + item, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// all 256 threads of every block, after its last share, which thread 0 has left: block of `size` in `group` of `groups` (size 1: no words of their
+// own); sh: 257 floats of LDS that nobody reads any more
+__device__ __forceinline__ void sum_shares(const BlockSum &q, int items, int size, int group, int groups, float *sh)
+{
+    if (threadIdx.x == 0) {
+        __builtin_amdgcn_s_waitcnt(0);   // the shares are in memory
+        bool last = size == 1 || __hip_atomic_fetch_add(q.arrived + 1 + group, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned int)size - 1;
+        if (last) last = __hip_atomic_fetch_add(q.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned int)groups - 1;
+        sh[256] = last ? 1.0f : 0.0f;
+    }
+    __syncthreads();
+    if (sh[256] == 0.0f) return;
+    float v = 0.0f;
+    for (int i = threadIdx.x; i < items; i += 256) v += __hip_atomic_load(q.part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    sh[threadIdx.x] = v;
+    __syncthreads();
+    for (int h = 128; h >= 1; h >>= 1) {
+        if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        if (q.out_bf16) *static_cast<bf16_t *>(q.out) = f32_to_bf16(sh[0]);
+        else *static_cast<float *>(q.out) = sh[0];
+    }
+}
+
 #ifdef RDB_STAMPS
 #ifndef RDB_STAMP_KERNEL_ID
 #define RDB_STAMP_KERNEL_ID 0

@@ -19,7 +19,7 @@ int num_compute_units();   // of the current device (rdb_error.hip)
 // rdb_big.hip
 int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);
 int linear_rbias_big(void *dst, int64_t ld_dst, int64_t cols, const void *src, int64_t ld_src, int64_t contraction, uint32_t sR, uint32_t sK,
-                     const void *scale, const rdb_linear_desc *d, void *table, const void *other, int64_t ld_other, float *dot_part, int *tiles,
+                     const void *scale, const rdb_linear_desc *d, void *table, const void *other, int64_t ld_other, float *dot_part, void *dscale, int dscale_dtype,
                      int num_cus, hipStream_t s);
 
 constexpr int RB_BI = 64, RB_BT = 256, RB_BK = 64;
@@ -71,6 +71,7 @@ struct RBiasParams {
     // tile the accumulators as the lanes hold them, [wave][feature block][token block][quad][lane][4]
     int ranges, range_stages;
     float *part;
+    BlockSum dscale;   // of the launch that adds them up, a group per tile; RB_PART clears its counters (NULL: none)
 };
 enum { RB_ADD = 0, RB_ADD_DOT = 1, RB_PART = 2 };
 constexpr int RB_TILE = RB_BI * RB_BT;
@@ -100,6 +101,10 @@ template <int MODE> __global__ __launch_bounds__(256, 2) void rbias_add_kernel(R
     GlobalOperand<RB_BT, RB_BK, K_CONT> opdy = {p.dy, p.lddy, tok0, p.tokens, min(p.out_f, s_end * RB_BK), (int64_t)(p.tokens - 1) * p.lddy + p.out_f};
     gemm_mainloop<RB_BI, RB_BT, RB_BK, 1, 2, 1>(acc, lds, opr, opdy, s_begin * RB_BK, s_end - s_begin);
     if constexpr (MODE == RB_PART) {
+        if (p.dscale.arrived && range == 0 && threadIdx.x == 0) {
+            p.dscale.arrived[1 + w] = 0u;
+            if (w == 0) *p.dscale.arrived = 0u;
+        }
         constexpr float unit = 4.656612873077392578125e-10f;
         f32x4 *dst = reinterpret_cast<f32x4 *>(p.part + (int64_t)item * RB_TILE) + threadIdx.x / 64 * (MI * NI * 4 * 64) + threadIdx.x % 64;
 #pragma unroll
@@ -229,12 +234,13 @@ template <bool DOT> __global__ __launch_bounds__(256) void rbias_sum_ranges_kern
         *reinterpret_cast<f32x4 *>(p.dx + at) = nw.f4;
     }
     if (DOT) {   // lanes, then waves, in a fixed order
-        __shared__ float wsum[4];
+        __shared__ float wsum[4], sh[257];
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) dot += __shfl_xor(dot, off, 64);
         if ((t & 63) == 0) wsum[t >> 6] = dot;
         __syncthreads();
-        if (t == 0) p.dot_part[blockIdx.x] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+        if (t == 0) leave_share(p.dscale, blockIdx.x, (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]));
+        sum_shares(p.dscale, gridDim.x, SUBS, w, p.tiles_i * p.tiles_t, sh);
     }
 }
 
@@ -489,19 +495,20 @@ static void rb_ranges(const rdb_linear_desc *d, int64_t cols, int num_cus, int &
     }
     range_stages = (int)per(ranges);
 }
-// Scratch for the ranges' sums (0: one range), and for one float per block that adds them up
+// Scratch for the ranges' sums (0: one range), for one float per block that adds them up, and for their counts
 static int64_t rb_part_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus)
 {
     int ranges, range_stages;
     rb_ranges(d, cols, num_cus, ranges, range_stages);
-    return ranges > 1 ? rb_tiles(d, cols) * (ranges * (RB_TILE * 4ll) + RB_BT / 32 * 4ll) : 0;
+    return ranges > 1 ? rb_tiles(d, cols) * (ranges * (RB_TILE * 4ll) + RB_BT / 32 * 4ll + 4) + 4 : 0;
 }
 
-// What a call uses beyond the tiles' shares of the scale's gradient: R for the 256-wide tiles, or the ranges' sums.
+// What a call uses beyond the tiles' shares of the scale's gradient: R for the 256-wide tiles and a
+// word that their blocks count in, or the ranges' sums.
 int64_t rbias_scratch_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus)
 {
     const int64_t table = rbias_big_table_bytes(d, cols, num_cus);
-    return table > 0 ? table : rb_part_bytes(d, cols, num_cus);
+    return table > 0 ? table + 256 : rb_part_bytes(d, cols, num_cus);
 }
 
 // other / dot_part / dscale: NULL, or the matrix the product is reduced against, room for one float per tile, and where the sum goes;
@@ -533,30 +540,25 @@ static int rbias_add(void *dst, int64_t ld_dst, int64_t cols, const void *src, i
     p.dot_part = dot_part;
     if (other && (ld_other % 8 || ((uintptr_t)other & 15) || d->tokens * ld_other >= (1ll << 29) || !dot_part || !dscale)) return RDB_E_UNSUPPORTED;
     const int64_t need = table ? rbias_big_table_bytes(d, cols, num_compute_units()) : 0;
-    if (need > 0 && table_bytes >= need && !((uintptr_t)table & 15) && (!other || cdiv(cols, 256) * cdiv(d->tokens, 128) <= linear_dx_rbias_dot_floats(d))) {
-        int tiles = 0;
-        if (int rc = linear_rbias_big(dst, ld_dst, cols, src, ld_src, contraction, sR, sK, scale_bias, d, table, other, ld_other, dot_part, &tiles,
-                                      num_compute_units(), s))
-            return rc;
-        if (!other) return RDB_OK;
-        return launch_rbias_sum(dscale, dscale_dtype, dot_part, tiles, s);
-    }
+    if (need > 0 && table_bytes >= need + (other ? 4 : 0) && !((uintptr_t)table & 15) && (!other || cdiv(cols, 256) * cdiv(d->tokens, 128) <= linear_dx_rbias_dot_floats(d)))
+        return linear_rbias_big(dst, ld_dst, cols, src, ld_src, contraction, sR, sK, scale_bias, d, table, other, ld_other, dot_part, dscale, dscale_dtype,
+                                num_compute_units(), s);
     size_t smem = engine_smem<RB_BI, RB_BT, RB_BK, K_CONT, K_CONT>();
     const int tiles = p.tiles_i * p.tiles_t;
     const int64_t part = table && !((uintptr_t)table & 15) ? rb_part_bytes(d, cols, num_compute_units()) : 0;
     if (part > 0 && table_bytes >= part) {
         rb_ranges(d, cols, num_compute_units(), p.ranges, p.range_stages);
         p.part = static_cast<float *>(table);
-        p.dot_part = p.part + (int64_t)tiles * p.ranges * RB_TILE;
-        if (int rc = launch_engine(rbias_add_kernel<RB_PART>, p, tiles * p.ranges, smem, s, "rbias_add_kernel<part>")) return rc;
         const int blocks = tiles * (RB_BT / 32);
+        float *const dots = p.part + (int64_t)tiles * p.ranges * RB_TILE;
+        p.dscale = {dots, other ? reinterpret_cast<unsigned int *>(dots + blocks) : nullptr, dscale, dscale_dtype == RDB_BF16};
+        if (int rc = launch_engine(rbias_add_kernel<RB_PART>, p, tiles * p.ranges, smem, s, "rbias_add_kernel<part>")) return rc;
         if (!other) {
             rbias_sum_ranges_kernel<false><<<blocks, 256, 0, s>>>(p);
             return check_launch("rbias_sum_ranges_kernel");
         }
         rbias_sum_ranges_kernel<true><<<blocks, 256, 0, s>>>(p);
-        if (int rc = check_launch("rbias_sum_ranges_kernel<dot>")) return rc;
-        return launch_rbias_sum(dscale, dscale_dtype, p.dot_part, blocks, s);
+        return check_launch("rbias_sum_ranges_kernel<dot>");
     }
     // tiles of 512 tokens when they give at least every other compute unit a block (half the hashing per product: measured
     // ahead from there on; 8192 tokens x 768 features, contraction 3072: 83 -> 67 us), tiles of 256 tokens otherwise

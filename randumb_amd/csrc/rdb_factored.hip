@@ -44,11 +44,13 @@ struct ZParams {
     unsigned long long sync_tag;
     // The contraction is added up in `ranges` ranges of range_stages stages of 64 features, range by range, whoever computes them.
     // part == NULL: every block runs its tile's ranges one after the other.  Otherwise the grid holds a block per tile and range,
-    // range by range; the blocks of the last range of a tile wait for the others' sums.  A token tile's sums lie in its own
-    // rows of y, which nobody writes before they have been read (a multiplying block waits for all of its tokens' z):
-    // [coefficient tile][range][token of the tile][32] floats, and behind them, at the end of the rows, a tag for each.
+    // range by range; the blocks of the last range of a tile wait for the others' sums.  A token tile's sums lie in its tokens' rows, of
+    // part_row bytes each, of y, which nobody writes before they have been read (a multiplying block waits for all of its tokens' z),
+    // or behind the state: [coefficient tile][range][token of the tile][32] floats, and behind them, at the end of the rows, a tag for each.
     int ranges, range_stages;
     char *part;
+    int64_t part_row;
+    int part_stays;   // nothing is written over the tags before the next launch
     SyncWait sync_wait;
     // C's transposition: by the projecting blocks, after their tiles, or (c_blocks > 0) by that many blocks behind the z_grid projecting ones
     int z_grid, c_blocks;
@@ -135,6 +137,13 @@ template <bool RANGES> __device__ __forceinline__ void z_block(const ZParams &p,
     // before this tile is touched.
     if (p.sync && t == 0 && (!part || my_range == p.ranges - 1))
         __hip_atomic_store(p.sync + (int64_t)(w / p.tiles_m) * (p.tiles_m + 1) + w % p.tiles_m, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // ... and a range's tag, which is still there where y does not take its place
+    auto range_tags = [&]() {
+        return reinterpret_cast<unsigned long long *>(p.part + (int64_t)(tok0 + min(KZ_BT, p.tokens - tok0)) * p.part_row) -
+               (int64_t)(p.tiles_m - w % p.tiles_m) * (p.ranges - 1);
+    };
+    if (part && p.part_stays && my_range < p.ranges - 1 && t == 0)
+        __hip_atomic_store(range_tags() + my_range, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     RDB_STAMP(0);
     typedef OperandTile<KZ_BM, F_BK, K_CONT> TN;   // noise tile: rows = coefficients, contraction = input features
     typedef OperandTile<KZ_BT, F_BK, K_CONT> TX;   // x tile: rows = tokens
@@ -222,9 +231,8 @@ template <bool RANGES> __device__ __forceinline__ void z_block(const ZParams &p,
     __syncthreads();   // the last stage's fragment reads are done: the tile buffers may be reused
     if (part) {
         const int rows = min(KZ_BT, p.tokens - tok0), others = p.ranges - 1, mt = w % p.tiles_m;
-        char *base = p.part + (int64_t)tok0 * p.out_f * 2;
-        unsigned long long *tags = reinterpret_cast<unsigned long long *>(base + (int64_t)rows * p.out_f * 2) - (int64_t)p.tiles_m * others + mt * others;
-        const __amdgpu_buffer_rsrc_t rs_p = __builtin_amdgcn_make_buffer_rsrc(base, 0, p.tiles_m * others * rows * 128, 0x00020000);
+        unsigned long long *tags = range_tags();
+        const __amdgpu_buffer_rsrc_t rs_p = __builtin_amdgcn_make_buffer_rsrc(p.part + (int64_t)tok0 * p.part_row, 0, p.tiles_m * others * rows * 128, 0x00020000);
         const int row = wave * 32 + (lane & 31);
         auto at = [&](int rg, int jq) { return row < rows ? (uint32_t)(((mt * others + rg) * rows + row) * 128 + (8 * jq + 4 * (lane >> 5)) * 4) : BUFFER_OOB; };
         if (my_range < others) {
@@ -255,6 +263,7 @@ template <bool RANGES> __device__ __forceinline__ void z_block(const ZParams &p,
             const bool there = await_tags(tags, others, p.sync_tag, p.sync_wait);
             if (!there && p.sync)
                 mark_gone(reinterpret_cast<unsigned int *>(p.sync + (int64_t)(w / p.tiles_m) * (p.tiles_m + 1) + p.tiles_m) + 1, p.sync_tag);
+            if (there && p.part_stays && lane < others) __hip_atomic_store(tags + lane, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // a replay carries the same tag
             if (lane == 0) *verdict = there ? 1 : 0;
         }
         __syncthreads();
@@ -425,8 +434,6 @@ static bool factored_shape_ok(const rdb_linear_desc *d) { return proj_layout(d).
 static bool cheaper_factored(const rdb_linear_desc *d) { return d->k * (d->in_f + d->out_f) < 16 * d->in_f * d->out_f; }
 static bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
-int64_t linear_projection_bytes(const rdb_linear_desc *d) { return proj_layout(d).bytes; }
-
 static bf16_t *state_piece(const void *state, int64_t off) { return reinterpret_cast<bf16_t *>(static_cast<char *>(const_cast<void *>(state)) + off); }
 
 // Fills the coefficient-gradient parameters that name the projection state's pieces.
@@ -447,18 +454,35 @@ int linear_fwd_projected(void *y, int64_t ldy, const void *state, const void *co
 // Ranges of the projection's contraction.  A tile's block walks over all of in_f, half a microsecond per 64 features: with fewer
 // tiles than compute units the others stand idle meanwhile (2000 tokens x 4096 features, k = 256: 64 tiles of 64 stages).  So as
 // many ranges as leave a unit for every block, of at least KZ_MIN_STAGES stages: below that the wait for the others' sums and
-// fetching them (some 4 us) costs what the shorter loop saves.  The sums need (ranges - 1) * kpad * 4 bytes of a token's out_f * 2.
-// The numbers depend on the layer alone, so that the same sums in the same order come out wherever they are computed.
+// fetching them (some 4 us) costs what the shorter loop saves.  The numbers depend on the layer alone, so that the same sums in the same
+// order come out wherever they are computed.  The sums need (ranges - 1) * kpad * 4 bytes of a token's out_f * 2 in y; layers too narrow for that have
+// room behind their state, 9 MB at most (ranges times tiles are at most the compute units, a sum 32 KB).  With as many ranges as y holds instead: 640
+// tokens x 3400 -> 696, k = 264, one range: 28.6 us, now 20.4; 200 x 8000 -> 1000, k = 400: 39.2, 24.2; 700 x 4000 -> 400, k = 200: 42.6, 26.4; 1056 x
+// 3072 -> 768, k = 240, two ranges: 28.6, 25.5; 2048 x 3072 -> 768, k = 256: 27.8, 24.8.
 constexpr int KZ_MIN_STAGES = 8, KZ_MAX_RANGES = 16;
 static void z_ranges(const rdb_linear_desc *d, int tiles, int &ranges, int &range_stages)
 {
-    const int nstage = (int)cdiv(d->in_f, F_BK), kpad = (int)cdiv(d->k, 64) * 64;
+    const int nstage = (int)cdiv(d->in_f, F_BK);
     int64_t r = std::min<int64_t>(std::min<int64_t>(num_compute_units() / tiles, nstage / KZ_MIN_STAGES), KZ_MAX_RANGES);
-    r = std::min<int64_t>(r, 1 + (d->out_f * 2 - 64) / (kpad * 4 + kpad / 4));
     if (r < 1) r = 1;
     range_stages = (int)cdiv(nstage, r);
     range_stages += range_stages & 1;   // the stages alternate between two buffers, beginning with the first
     ranges = (int)cdiv(nstage, range_stages);
+}
+// bytes of a token's share of the ranges' sums and their tags where y's row does not hold them, else 0
+static int64_t z_part_row(const rdb_linear_desc *d, int ranges)
+{
+    const int64_t kpad = cdiv(d->k, 64) * 64, row = (ranges - 1) * (kpad * 4 + kpad / 4);
+    return row + 64 > d->out_f * 2 ? row : 0;
+}
+// the state, and behind it room for the ranges' sums of layers whose y has none
+int64_t linear_projection_bytes(const rdb_linear_desc *d)
+{
+    const ProjLayout L = proj_layout(d);
+    if (!L.ok) return L.bytes;
+    int ranges, range_stages;
+    z_ranges(d, (int)(L.kpad / KZ_BM * cdiv(d->tokens, KZ_BT)), ranges, range_stages);
+    return L.bytes + (ranges > 1 ? (d->tokens * z_part_row(d, ranges) + 255) / 256 * 256 : 0);
 }
 
 static bool fill_z_params(ZParams &p, void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d)
@@ -494,12 +518,22 @@ static bool fill_z_params(ZParams &p, void *state, const void *x, int64_t ldx, c
 }
 
 // Spreads the ranges of a split contraction over blocks of their own, with the sums on the way in y's rows (contiguous, not yet
-// written).  False when there is nothing to spread, or y is not the place.
+// written) or, where those are too short, behind the state.  False when there is nothing to spread, or y is not the place.
 static bool spread_ranges(ZParams &p, void *state, void *y, int64_t ldy, const rdb_linear_desc *d, int *rc)
 {
     *rc = RDB_OK;
-    if (p.ranges <= 1 || !y || ldy != d->out_f || !aligned16(y) || !one_launch_mode()) return false;
-    p.part = static_cast<char *>(y);
+    if (p.ranges <= 1 || !one_launch_mode()) return false;
+    if (const int64_t row = z_part_row(d, p.ranges)) {
+        p.part = static_cast<char *>(state) + proj_layout(d).bytes;
+        p.part_row = row;
+        p.part_stays = 1;
+    } else if (y && ldy == d->out_f && aligned16(y)) {
+        p.part = static_cast<char *>(y);
+        p.part_row = d->out_f * (int64_t)sizeof(bf16_t);
+        p.part_stays = 0;
+    } else {
+        return false;
+    }
     if (!p.sync_tag) p.sync_tag = next_sync_tag();
     p.sync_wait.err = reinterpret_cast<unsigned int *>(state) + 1;
     p.sync_wait.polls = SYNC_SPIN_LIMIT;

@@ -773,9 +773,8 @@ inline int64_t fg_chunk(int64_t K, int r)
     return r > 1 && (cdiv(K, chunk) != r || chunk < 64) ? 0 : chunk;
 }
 constexpr double FG_HOST_US = 3.8, FG_SHORT_US = 16.0;
-inline FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int max_ranges, bool groups4, double host_us = 0.0)
+inline FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int max_ranges, bool groups4, double host_us = 0.0, bool split = f32_split_mode() != 0)
 {
-    const bool split = f32_split_mode() != 0;
     const double out_mb = (double)M * N * 4e-6;
     FgPlan best = {128, 1, 1};
     double best_us = 1e30;

@@ -432,13 +432,15 @@ static int64_t vec_dcoef_workspace(const rdb_linear_desc *d)
 
 static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d);
 namespace rdb {
+int64_t linear_kept_f32_z_bytes(const rdb_linear_desc *d);   // rdb_f32.hip
 int64_t linear_bwd_kept_f32_workspace(const rdb_linear_desc *d, int num_cus);   // rdb_f32.hip
 }
 
+static bool kept_layer(const rdb_linear_desc *d);
 extern "C" int64_t rdb_linear_workspace_bytes(int op, const rdb_linear_desc *d)
 {
     if (!d) return 0;
-    if (op == RDB_OP_LINEAR_BWD_KEPT) return rdb_linear_kept_bytes(d) ? linear_bwd_kept_f32_workspace(d, num_compute_units()) : 0;
+    if (op == RDB_OP_LINEAR_BWD_KEPT) return kept_layer(d) ? linear_bwd_kept_f32_workspace(d, num_compute_units()) : 0;
     int64_t need = linear_workspace_bytes_main(op, d);
     if (d->algo == RDB_ALGO_AUTO && d->act_dtype == RDB_BF16 && d->coef_rows != 0 &&
         (op == RDB_OP_LINEAR_FWD || op == RDB_OP_LINEAR_BWD_DX || op == RDB_OP_LINEAR_BWD_DCOEF)) {
@@ -1292,17 +1294,17 @@ int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, fl
                         int64_t workspace_bytes, hipStream_t s);
 }
 
-extern "C" int64_t rdb_linear_kept_bytes(const rdb_linear_desc *d)
+static bool kept_layer(const rdb_linear_desc *d)
 {
-    if (check_desc("rdb_linear_kept_bytes", d) || rdb_linear_projection_preferred(d)) return 0;
-    return linear_kept_f32_bytes(d);
+    return !check_desc("rdb_linear_kept_bytes", d) && !rdb_linear_projection_preferred(d) && linear_kept_f32_z_bytes(d) > 0;
 }
+extern "C" int64_t rdb_linear_kept_bytes(const rdb_linear_desc *d) { return kept_layer(d) ? linear_kept_f32_bytes(d) : 0; }
 
 static int fwd_kept(const char *who, void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
                     const rdb_pseudo_bias *values, const rdb_linear_desc *d, void *stream)
 {
     if (int rc = check_desc(who, d)) return rc;
-    if (!rdb_linear_kept_bytes(d)) return set_error(RDB_E_UNSUPPORTED, "%s: a layer of which nothing is kept (rdb_linear_kept_bytes)", who);
+    if (!kept_layer(d)) return set_error(RDB_E_UNSUPPORTED, "%s: a layer of which nothing is kept (rdb_linear_kept_bytes)", who);
     if (!y || !kept || !x || !coef) return set_error(RDB_E_NULL, "%s: y, kept, x or coef is NULL", who);
     if (ldx < d->in_f || ldy < d->out_f) return set_error(RDB_E_SHAPE, "%s: leading dimension smaller than the row", who);
     if (values) {
@@ -1333,7 +1335,7 @@ extern "C" int rdb_linear_bwd_kept(void *dx, int64_t lddx, void *dcoef, int dcoe
                                    int64_t workspace_bytes, void *stream)
 {
     if (int rc = check_desc("rdb_linear_bwd_kept", d)) return rc;
-    if (!rdb_linear_kept_bytes(d)) return set_error(RDB_E_UNSUPPORTED, "rdb_linear_bwd_kept: a layer of which nothing is kept (rdb_linear_kept_bytes)");
+    if (!kept_layer(d)) return set_error(RDB_E_UNSUPPORTED, "rdb_linear_bwd_kept: a layer of which nothing is kept (rdb_linear_kept_bytes)");
     if (!dy || (dx && !coef) || (dcoef && !kept) || (d_scale_bias && (!x || !scale_bias)))
         return set_error(RDB_E_NULL, "rdb_linear_bwd_kept: dy, x, kept, coef or scale_bias is NULL");
     if (lddy < d->out_f || (dx && lddx < d->in_f) || (d_scale_bias && ldx < d->in_f))

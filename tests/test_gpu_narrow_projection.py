@@ -41,3 +41,43 @@ def test_narrow_layers(T, in_f, out_f, k):
         assert torch.equal(hip.linear_fwd_projected(alone, c, in_f, 5), want[i]), i
         assert torch.equal(hip.linear_project_fwd(xs[i], c, 5)[0], want[i])
     hip.sync_check()
+
+
+# fp32 sums: odd sizes in bf16, and fp32; one token more than a tile, several ranges, y of one column
+@pytest.mark.parametrize("T,in_f,out_f,k,dtype", [(492, 3184, 273, 118, torch.bfloat16), (129, 1027, 1, 20, torch.bfloat16), (433, 3320, 96, 144, torch.float32),
+                                                  (65, 4000, 33, 257, torch.float32)])
+@pytest.mark.parametrize("split", [1, 0])
+def test_narrow_layers_in_fp32_sums(T, in_f, out_f, k, dtype, split):
+    import ctypes
+
+    from randumb_amd import _lib, hip
+
+    print(f"case narrow kept T={T} in={in_f} out={out_f} k={k} {dtype} split={split}", flush=True)
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator().manual_seed(T)
+    x, c = torch.randn(T, in_f, generator=g).to(dtype).cuda(), (torch.randn(out_f, k, generator=g) / k ** 0.5).to(dtype).cuda()
+    ref = ctypes.byref(hip._desc(T, in_f, out_f, c, in_f, 1, 5, dtype, 0))
+    N = hip.sq5_fill_2d(in_f, k, 5).double()
+    z = x.double() @ N
+    want = z @ c.double().t()
+    calls = [("kept", lib.rdb_linear_kept_bytes(ref), 0)] + ([("state", lib.rdb_linear_projection_bytes(ref), 256)] if dtype is torch.float32 else [])
+    assert max(n for _, n, _ in calls) > 256 + (T * k * 4 + 255) // 256 * 256   # room for ranges
+    for what, n, at in calls:
+        if n == 0:
+            continue
+        kept = torch.full((n + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+        y = torch.full((T + 1, out_f), 7.0, dtype=dtype, device="cuda")
+        before = lib.rdb_set_f32_split(split)   # asked for after the buffer's size
+        try:
+            if what == "kept":
+                rc = lib.rdb_linear_fwd_kept(y.data_ptr(), out_f, kept.data_ptr(), x.data_ptr(), in_f, c.data_ptr(), None, None, ref, stream)
+            else:
+                rc = lib.rdb_linear_project_fwd(y.data_ptr(), out_f, kept.data_ptr(), x.data_ptr(), in_f, c.data_ptr(), None, ref, stream)
+        finally:
+            lib.rdb_set_f32_split(before)
+        assert rc == 0 and bool((kept[n:] == 0x5A).all()) and bool((y[T] == 7.0).all())
+        got = kept[at:at + T * k * 4].view(torch.float32).view(T, k).double()
+        assert float((got - z).norm() / z.norm()) < 2e-6   # fp32 sums of products of fp32 accuracy
+        # y rounded once: to bf16 2^-9 at most
+        assert float((y[:T].double() - want).norm() / want.norm()) < (2.0 ** -9 if dtype is torch.bfloat16 else 4e-6)
+    hip.sync_check()

@@ -213,6 +213,13 @@ static int fg_launch_pair_ranges(FgProduct t, int t_room, float *t_part, int64_t
     return fg_launch_sums(sum[0], sum[1], s);
 }
 
+// What z's launch of sums counts for on the host: nothing where the step's products, z, y, t, dC and dx at 1.16 PFLOP/s, take 40 us and more (with as much
+// again for what they wait, the kernels then outlast the host's 60 to 70: 2859 tokens x 584 -> 7920, k = 208, step 219 us, 222 with z in one range).
+static double z_host_us(const rdb_linear_desc *d)
+{
+    const double parts = d->act_dtype == RDB_BF16 ? 3.0 : 6.0;   // bf16 products per product
+    return parts * 2.0 * d->tokens * d->k * (2.0 * d->in_f + 3.0 * d->out_f) / 1.16e9 < 40.0 ? FG_HOST_US : 0.0;
+}
 // z[T x k] = src[T x in_f] . N^T; the partial matrices of its ranges go to `part` (room for max_ranges of them, up256(T k 4)
 // bytes apart; NULL: right behind z, as many as there is room for)
 static int fg_project(float *z, const float *x, int64_t ldx, const rdb_linear_desc *d, int num_cus, hipStream_t s, float *part = nullptr,
@@ -223,7 +230,7 @@ static int fg_project(float *z, const float *x, int64_t ldx, const rdb_linear_de
     q.values = values;
     const int64_t zt = up256(d->tokens * d->k * 4) / 4;
     return fg_launch_ranges<FG_KCONT, FG_NOISE_M>(q, std::max(1, std::min(z_room(d, num_cus), max_ranges)), part ? part : z + zt, zt, num_cus, s,
-                                                  "f32_gemm_kernel (z = x . N^T)", FG_HOST_US);
+                                                  "f32_gemm_kernel (z = x . N^T)", z_host_us(d));
 }
 
 // Where the forward pass puts the partial matrices of z's ranges: into y, which is written last, or, where y holds less than a third of those that pay, behind
@@ -237,7 +244,7 @@ static int64_t z_behind(const rdb_linear_desc *d)
     const int64_t zt = up256(d->tokens * d->k * 4), in_y = std::max<int64_t>(1, d->tokens * d->out_f * fg_es(d->act_dtype) / zt);
     if (z_room(d, num_cus) < 3 * in_y) return 0;
     // by the layer alone, whatever products are asked for (rdb_set_f32_split): what is kept may be larger than they need, never smaller
-    const int want = fg_plan(d->tokens, d->k, d->in_f, num_cus, std::max(1, z_room(d, num_cus)), FgGroups<FG_KCONT, FG_NOISE_M>::four, FG_HOST_US, true).ranges;
+    const int want = fg_plan(d->tokens, d->k, d->in_f, num_cus, std::max(1, z_room(d, num_cus)), FgGroups<FG_KCONT, FG_NOISE_M>::four, z_host_us(d), true).ranges;
     return want >= 3 * in_y ? want * zt : 0;
 }
 // z into `z`, y (or NULL) to come, with what z_behind says behind z

@@ -756,7 +756,10 @@ inline FgPlan fg_room(int64_t M, int64_t N, int64_t K, int num_cus, int64_t min_
 // share a unit take `unit` us of its throughput each, a launch `base` us and every further round of blocks 2.6; outputs leave at 4.8 TB/s; adding ranges up is one more
 // launch, whose 14 TB/s say that the partial matrices come back out of the caches.  `host_us`: what that launch counts
 // for besides: a step whose kernels are shorter than the host's work on it (50 to 70 us for a layer) pays for the launch as well, so where the
-// product is short (FG_SHORT_US) ranges have to gain more than both.  `resident`, the groups that take turns on a unit's
+// product is short (FG_SHORT_US, and less and less up to FG_LONG_US) ranges have to gain more than both, and 4 % where it
+// is long: a product that fills the chip a little better slows the kernels beside it, which share its power (a vector-coef step of 696 tokens x 856
+// -> 3069, k = 74: y 41.7 -> 39.1 us in three ranges, 3.7 % by the model, the hashing kernels 190 -> 204; dW of 1024 x 768 -> 3072, 4.7 %: 45.5 -> 41.0 and
+// the others as they were).  `resident`, the groups that take turns on a unit's
 // time, was fitted with the others and is not what registers and LDS leave room for.  The products measured had fp32 matrices; a
 // side that comes from a bf16 matrix takes less LDS and fewer registers (four to seven blocks of 256 threads fit a unit), and hashing
 // is not told apart: for those the constants are what they are for fp32.
@@ -772,26 +775,38 @@ inline int64_t fg_chunk(int64_t K, int r)
     const int64_t chunk = cdiv(cdiv(K, r), FG_BK) * FG_BK;
     return r > 1 && (cdiv(K, chunk) != r || chunk < 64) ? 0 : chunk;
 }
-constexpr double FG_HOST_US = 3.8, FG_SHORT_US = 16.0;
+constexpr double FG_HOST_US = 3.8, FG_SHORT_US = 16.0, FG_LONG_US = 24.0, FG_HEAT = 0.04;
 inline FgPlan fg_plan(int64_t M, int64_t N, int64_t K, int num_cus, int max_ranges, bool groups4, double host_us = 0.0, bool split = f32_split_mode() != 0)
 {
     const double out_mb = (double)M * N * 4e-6;
     FgPlan best = {128, 1, 1};
     double best_us = 1e30;
-    for (const FgKind &kd : FG_KINDS) {
-        if (kd.groups > 1 && (!split || (kd.groups == 4 && !groups4))) continue;
-        const int64_t tiles = cdiv(M, kd.bm) * cdiv(N, FG_BN);
-        for (int r = 1; r <= max_ranges; ++r) {
-            const int64_t chunk = fg_chunk(K, r);
-            if (!chunk) continue;
-            const int64_t per_cu = cdiv(tiles * r, num_cus), stages = cdiv(chunk / FG_BK, kd.groups);
-            const int64_t rounds = cdiv(per_cu, kd.resident);
-            double us = kd.base + 2.6 * (rounds - 1) + stages * (rounds * kd.chain + per_cu * kd.groups * kd.unit) + out_mb * r * 0.21 +
-                              (r > 1 ? 4.2 + out_mb * r * 0.07 : 0.0);
-            if (r > 1 && us < FG_SHORT_US) us += host_us;
+    // the ranges that fg_chunk allows and the stages of each, once for all kinds: a step makes five plans, and this is host time (1.2 us a plan of 32
+    // ranges with a chunk and three 64-bit divisions per range and kind, 0.4 so)
+    constexpr uint32_t CAP = 64;
+    uint32_t count = 0, ranges[CAP], stages_of[CAP];
+    const uint32_t all = (uint32_t)cdiv(K, FG_BK), most = (uint32_t)(max_ranges < (int)CAP ? max_ranges : (int)CAP);
+    for (uint32_t r = 1; r <= most; ++r) {
+        const uint32_t n = (all + r - 1) / r;
+        if (r > 1 && n < 4) break;
+        if (r > 1 && (all + n - 1) / n != r) continue;
+        ranges[count] = r;
+        stages_of[count++] = n;
+    }
+    auto tiles = [&](int bm) { return (uint32_t)std::min<int64_t>(cdiv(M, bm) * cdiv(N, FG_BN), 1 << 25); };
+    const uint32_t t128 = tiles(128), t64 = tiles(64);
+    for (uint32_t i = 0; i < count; ++i) {
+        const uint32_t r = ranges[i];
+        const double more = r > 1 ? 4.2 + out_mb * r * 0.28 : out_mb * 0.21;
+        for (const FgKind &kd : FG_KINDS) {
+            if (kd.groups > 1 && (!split || (kd.groups == 4 && !groups4))) continue;
+            const uint32_t per_cu = ((kd.bm == 128 ? t128 : t64) * r + (uint32_t)num_cus - 1) / (uint32_t)num_cus, rounds = (per_cu + (uint32_t)kd.resident - 1) / (uint32_t)kd.resident;
+            const uint32_t stages = (stages_of[i] + (uint32_t)kd.groups - 1) / (uint32_t)kd.groups;
+            double us = kd.base + 2.6 * (rounds - 1) + stages * (rounds * kd.chain + per_cu * kd.groups * kd.unit) + more;
+            if (r > 1 && host_us > 0.0) us += std::max(FG_HEAT * us, us < FG_SHORT_US ? host_us : host_us * (FG_LONG_US - us) / (FG_LONG_US - FG_SHORT_US));
             if (us < best_us) {
                 best_us = us;
-                best = {kd.bm, r, kd.groups};
+                best = {kd.bm, (int)r, kd.groups};
             }
         }
     }

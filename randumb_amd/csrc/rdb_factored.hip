@@ -475,15 +475,16 @@ static int64_t z_part_row(const rdb_linear_desc *d, int ranges)
     const int64_t kpad = cdiv(d->k, 64) * 64, row = (ranges - 1) * (kpad * 4 + kpad / 4);
     return row + 64 > d->out_f * 2 ? row : 0;
 }
-// the state, and behind it room for the ranges' sums of layers whose y has none
-int64_t linear_projection_bytes(const rdb_linear_desc *d)
+// the state, and behind it room for the ranges' sums of layers whose y has none, which a transient state may do without
+int64_t linear_projection_extra(const rdb_linear_desc *d)
 {
     const ProjLayout L = proj_layout(d);
-    if (!L.ok) return L.bytes;
+    if (!L.ok) return 0;
     int ranges, range_stages;
     z_ranges(d, (int)(L.kpad / KZ_BM * cdiv(d->tokens, KZ_BT)), ranges, range_stages);
-    return L.bytes + (ranges > 1 ? (d->tokens * z_part_row(d, ranges) + 255) / 256 * 256 : 0);
+    return ranges > 1 ? (d->tokens * z_part_row(d, ranges) + 255) / 256 * 256 : 0;
 }
+int64_t linear_projection_bytes(const rdb_linear_desc *d) { return proj_layout(d).bytes + linear_projection_extra(d); }
 
 static bool fill_z_params(ZParams &p, void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d)
 {
@@ -518,12 +519,13 @@ static bool fill_z_params(ZParams &p, void *state, const void *x, int64_t ldx, c
 }
 
 // Spreads the ranges of a split contraction over blocks of their own, with the sums on the way in y's rows (contiguous, not yet
-// written) or, where those are too short, behind the state.  False when there is nothing to spread, or y is not the place.
-static bool spread_ranges(ZParams &p, void *state, void *y, int64_t ldy, const rdb_linear_desc *d, int *rc)
+// written) or, where those are too short, behind the state (room: it has its extra bytes).  False when there is nothing to spread, or no place.
+static bool spread_ranges(ZParams &p, void *state, void *y, int64_t ldy, const rdb_linear_desc *d, bool room, int *rc)
 {
     *rc = RDB_OK;
     if (p.ranges <= 1 || !one_launch_mode()) return false;
     if (const int64_t row = z_part_row(d, p.ranges)) {
+        if (!room) return false;
         p.part = static_cast<char *>(state) + proj_layout(d).bytes;
         p.part_row = row;
         p.part_stays = 1;
@@ -554,12 +556,12 @@ static void set_z_grid(ZParams &p, int z_grid, int num_cus)
 static size_t z_smem() { return engine_smem<KZ_BM, KZ_BT, F_BK, K_CONT, K_CONT>(); }
 
 // y: NULL, or the rows of the forward product to come, free to hold sums on the way
-static int launch_z(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, hipStream_t s)
+static int launch_z(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, bool room, hipStream_t s)
 {
     ZParams p;
     int rc;
     if (!fill_z_params(p, state, x, ldx, coef, d)) return RDB_E_UNSUPPORTED;
-    const bool spread = spread_ranges(p, state, y, ldy, d, &rc);
+    const bool spread = spread_ranges(p, state, y, ldy, d, room, &rc);
     if (rc) return rc;
     const size_t smem = z_smem();
     const void *fn = p.ranges > 1 ? (const void *)factored_z_kernel<true> : (const void *)factored_z_kernel<false>;
@@ -571,21 +573,21 @@ static int launch_z(void *state, const void *x, int64_t ldx, const void *coef, v
     return check_launch("factored_z_kernel");
 }
 
-int linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, hipStream_t s)
+int linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, hipStream_t s, bool room)
 {
-    return launch_z(state, x, ldx, coef, nullptr, 0, d, s);
+    return launch_z(state, x, ldx, coef, nullptr, 0, d, room, s);
 }
 
 // The same ahead of a forward product: y's rows, contiguous and written last, hold N or sums on the way meanwhile.  With a contraction in
 // several ranges the 256-wide tiles' sums would differ from launch_z's (z_ranges).
 int linear_project_before(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, int num_cus,
-                          hipStream_t s)
+                          hipStream_t s, bool state_room)
 {
     ZParams p;
     if (!fill_z_params(p, state, x, ldx, coef, d)) return RDB_E_UNSUPPORTED;
     const int64_t room = ldy == d->out_f && p.ranges == 1 ? d->tokens * d->out_f * (int64_t)sizeof(bf16_t) : 0;
     const int rc = linear_z_big(state, x, ldx, coef, y, room, d, num_cus, s);
-    return rc != RDB_E_UNSUPPORTED ? rc : launch_z(state, x, ldx, coef, y, ldy, d, s);
+    return rc != RDB_E_UNSUPPORTED ? rc : launch_z(state, x, ldx, coef, y, ldy, d, state_room, s);
 }
 
 // The forward product's parameters when the contraction of a token fits in registers (z in fragment order); returns the
@@ -628,7 +630,7 @@ template <bool BIAS> static int launch_ys(const StParams &q, int items, hipStrea
 // contraction of a token fits in registers (k <= 256), otherwise in two.
 // polls: how long its multiplying blocks wait; fewer than SYNC_SPIN_LIMIT in a self-test only.
 int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, bool with_ct, const void *bias,
-                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls)
+                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls, bool room)
 {
     ZYParams p;
     if (!fill_z_params(p.z, state, x, ldx, with_ct ? coef : nullptr, d)) return RDB_E_UNSUPPORTED;
@@ -637,7 +639,7 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
         // check the second call's conditions before the first launch, so that a refusal leaves nothing half done
         if (d->coef_dtype != RDB_BF16 || ldy % 8 || !aligned16(y) || !aligned16(coef)) return RDB_E_UNSUPPORTED;
         if (((uintptr_t)bias & 7) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
-        if (int rc = linear_project_before(state, x, ldx, with_ct ? coef : nullptr, y, ldy, d, num_cus, s)) return rc;
+        if (int rc = linear_project_before(state, x, ldx, with_ct ? coef : nullptr, y, ldy, d, num_cus, s, room)) return rc;
         return linear_fwd_projected(y, ldy, state, coef, bias, d, num_cus, s);
     }
     const ProjLayout L = proj_layout(d);
@@ -650,7 +652,7 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
     p.y.sync_wait.polls = polls;
     if (int rc = sync_giveups_ptr(&p.y.sync_wait.giveups)) return rc;
     int rc;
-    const bool spread = spread_ranges(p.z, state, y, ldy, d, &rc);
+    const bool spread = spread_ranges(p.z, state, y, ldy, d, room, &rc);
     if (rc) return rc;
     set_z_grid(p.z, xcd_grid_size(p.z.tiles_m * p.z.tiles_t) * (spread ? p.z.ranges : 1), num_cus);
     return bias ? launch_zy<true>(p, y_items, s) : launch_zy<false>(p, y_items, s);
@@ -718,13 +720,13 @@ int linear_fwd_factored(void *y, int64_t ldy, const void *x, int64_t ldx, const 
                         const rdb_linear_desc *d, int num_cus, void *workspace, int64_t workspace_bytes, hipStream_t s)
 {
     if (scale_bias || d->coef_dtype != RDB_BF16 || !factored_shape_ok(d)) return RDB_E_UNSUPPORTED;  // the random-bias term is not low rank
-    if (!workspace || workspace_bytes < linear_projection_bytes(d)) return RDB_E_UNSUPPORTED;
+    if (!workspace || workspace_bytes < proj_layout(d).bytes) return RDB_E_UNSUPPORTED;
     if (d->algo == RDB_ALGO_AUTO && !cheaper_factored(d)) return RDB_E_UNSUPPORTED;
     // check everything before the first launch, so that a refusal leaves nothing half done
     if (d->tokens * ldx >= (1ll << 29) || ldx % 8 || ldy % 8 || !aligned16(x) || !aligned16(coef) || !aligned16(y) || !aligned16(workspace))
         return RDB_E_UNSUPPORTED;
     if (((uintptr_t)bias & 7) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
-    return linear_project_fwd(y, ldy, workspace, x, ldx, coef, false, bias, d, num_cus, s, SYNC_SPIN_LIMIT);
+    return linear_project_fwd(y, ldy, workspace, x, ldx, coef, false, bias, d, num_cus, s, SYNC_SPIN_LIMIT, workspace_bytes >= linear_projection_bytes(d));
 }
 
 // dC = dy^T . (x . N^T) with the projection state in the workspace; dcoef must have been zeroed on the same stream.
@@ -732,12 +734,12 @@ int linear_dcoef_factored(float *dcoef, const void *dy, int64_t lddy, const void
                           void *workspace, int64_t workspace_bytes, hipStream_t s)
 {
     if (!factored_shape_ok(d)) return RDB_E_UNSUPPORTED;
-    if (!workspace || workspace_bytes < linear_projection_bytes(d)) return RDB_E_UNSUPPORTED;
+    if (!workspace || workspace_bytes < proj_layout(d).bytes) return RDB_E_UNSUPPORTED;
     if (d->algo == RDB_ALGO_AUTO && !cheaper_factored(d)) return RDB_E_UNSUPPORTED;
     if (d->tokens * ldx >= (1ll << 29) || d->tokens * lddy >= (1ll << 29) || ldx % 8 || lddy % 8 || !aligned16(x) || !aligned16(dy) ||
         !aligned16(workspace))
         return RDB_E_UNSUPPORTED;
-    int rc = linear_project(workspace, x, ldx, nullptr, d, s);
+    int rc = linear_project(workspace, x, ldx, nullptr, d, s, workspace_bytes >= linear_projection_bytes(d));
     if (rc) return rc;
     return linear_dcoef_projected(dcoef, dy, lddy, workspace, d, num_cus, s);
 }

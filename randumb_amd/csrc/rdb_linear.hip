@@ -285,9 +285,10 @@ int linear_fwd_strip(void *y, int64_t ldy, const void *x, int64_t ldx, const voi
 
 // rdb_factored.hip
 int64_t linear_projection_bytes(const rdb_linear_desc *d);
-int linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, hipStream_t s);
+int64_t linear_projection_extra(const rdb_linear_desc *d);
+int linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, hipStream_t s, bool room = true);
 int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, bool with_ct, const void *bias,
-                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls = SYNC_SPIN_LIMIT);
+                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls = SYNC_SPIN_LIMIT, bool room = true);
 int linear_fwd_projected(void *y, int64_t ldy, const void *z, const void *coef, const void *bias, const rdb_linear_desc *d, int num_cus,
                          hipStream_t s);
 int linear_dcoef_projected(float *dcoef, const void *dy, int64_t lddy, const void *z, const rdb_linear_desc *d, int num_cus, hipStream_t s);
@@ -362,7 +363,7 @@ int linear_dx_rbias_add_dscale(void *dx, int64_t lddx, void *dscale, int dscale_
 int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);
 int64_t rbias_scratch_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);   // rdb_rbias.hip
 int linear_project_before(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, int num_cus,
-                          hipStream_t s);   // rdb_factored.hip
+                          hipStream_t s, bool state_room = true);   // rdb_factored.hip
 int linear_fwd_rbias_big(void *y, int64_t ldy, const void *x, int64_t ldx, const void *state, const void *coef, const void *scale, const void *bias,
                          const rdb_linear_desc *d, void *table, int num_cus, hipStream_t s);
 
@@ -916,7 +917,8 @@ extern "C" int rdb_linear_fwd_static(void *y, int64_t ldy, const void *x, int64_
 {
     int rc = check_desc("rdb_linear_fwd_static", d);
     if (rc) return rc;
-    const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_FWD, d);
+    int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_FWD, d);
+    if (need > RDB_STATIC_SCRATCH_BYTES && need == linear_projection_bytes(d)) need -= linear_projection_extra(d);   // goes without
     if (need > RDB_STATIC_SCRATCH_BYTES)
         return set_error(RDB_E_WORKSPACE, "rdb_linear_fwd_static: this layer's kernels use %lld bytes of scratch, the library's static scratch holds "
                                           "%lld: call rdb_linear_fwd with a workspace of the caller's", (long long)need, (long long)RDB_STATIC_SCRATCH_BYTES);

@@ -9,7 +9,9 @@ pytestmark = pytest.mark.gpu
 # k <= 256, one launch: one token, one range more than y would hold, sixteen ranges, several token tiles with a ragged last one; k > 256
 @pytest.mark.parametrize("T,in_f,out_f,k", [(1, 1032, 8, 8), (97, 2048, 64, 64), (257, 8192, 1024, 32), (600, 4104, 200, 160), (640, 3400, 696, 264), (255, 1544, 72, 520)])
 def test_narrow_layers(T, in_f, out_f, k):
-    from randumb_amd import hip
+    import ctypes
+
+    from randumb_amd import _lib, hip
 
     print(f"case narrow projection T={T} in={in_f} out={out_f} k={k}", flush=True)
     g = torch.Generator().manual_seed(T)
@@ -28,6 +30,17 @@ def test_narrow_layers(T, in_f, out_f, k):
         finally:
             hip.set_one_launch(old)
         want.append(y)
+    # a transient state without the room: y by the one-call form, from scratch of the caller's and, what fits there, the library's
+    lib, stream, y = _lib.load(), torch.cuda.current_stream().cuda_stream, torch.empty_like(want[0])
+    ref = ctypes.byref(hip._desc(T, in_f, out_f, c, in_f, 1, 5, torch.bfloat16, _lib.RDB_ALGO_FACTORED))
+    n = lib.rdb_linear_workspace_bytes(0, ref)
+    less = n - (T * 8 + 255) // 256 * 256
+    ws = torch.full((n,), 0x5A, dtype=torch.uint8, device="cuda")
+    for size in (n, less):
+        assert lib.rdb_linear_fwd(y.data_ptr(), out_f, xs[0].data_ptr(), in_f, c.data_ptr(), None, None, ref, ws.data_ptr(), size, stream) == 0
+        assert torch.equal(y, want[0])
+    assert lib.rdb_linear_fwd_static(y.data_ptr(), out_f, xs[0].data_ptr(), in_f, c.data_ptr(), None, None, ref, stream) == 0
+    assert torch.equal(y, want[0])
     x = xs[0].clone()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):

@@ -372,7 +372,7 @@ int rdb_linear_bwd_projected_to(void *dx, int64_t lddx, void *dcoef, int dcoef_d
 
 /* The projected form's counterpart for layers without a projection state (bf16 with sizes that are not multiples of 8, fp32
  * in the few-token regime; rdb_linear_kept_bytes says how much, 0: none, use the calls above): the forward pass leaves
- * z = x . N^T (fp32, [tokens x k] row-major) in `kept`, 16-byte aligned, and the backward pass starts from it.  scale_bias as
+ * z = x . N^T (fp32, [tokens x k] row-major, and behind it scratch of the call's own) in `kept`, 16-byte aligned, and the backward pass starts from it.  scale_bias as
  * in rdb_linear_fwd.  rdb_linear_bwd_kept: dx, dcoef (dcoef_dtype RDB_F32 or RDB_BF16) and d_scale_bias (fp32) are
  * overwritten, NULL where not wanted; x is read for d_scale_bias only; a workspace of
  * rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_KEPT, desc) bytes.  Sums in a fixed order. */

@@ -468,6 +468,39 @@ int64_t linear_bwd_kept_f32_workspace(const rdb_linear_desc *d, int num_cus)
            up256(cdiv(d->tokens, 64) * cdiv(std::max(d->in_f, d->out_f), FG_BN) * 4);
 }
 
+// dx += s * (the ranges' sums of dy . R, [rows x cols] each, `stride` floats apart, added in range order), all in bf16 but the sums; dots: NULL, or a
+// value per block, its share of their product with x.  One element a thread and turn: rows are of any length.
+__global__ __launch_bounds__(256) void f32_rbias_sum_kernel(bf16_t *__restrict__ dx, int64_t lddx, const float *__restrict__ part, int64_t stride, int ranges,
+                                                            const bf16_t *__restrict__ scale, const bf16_t *__restrict__ x, int64_t ldx, float *__restrict__ dots,
+                                                            uint32_t n, uint32_t cols)
+{
+    const float s = bf16_to_f32(*scale);
+    float dot = 0.0f;
+    for (uint32_t e = blockIdx.x * 256u + threadIdx.x; e < n; e += gridDim.x * 256u) {
+        const uint32_t row = e / cols, col = e - row * cols;
+        bf16_t *const to = dx + row * lddx + col;
+        const float old = bf16_to_f32(*to), other = dots ? bf16_to_f32(x[row * ldx + col]) : 0.0f;
+        float v = part[e];
+        for (int r0 = 1; r0 < ranges; r0 += 4) {   // four ranges' loads in flight
+            float u[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) u[j] = part[min(r0 + j, ranges - 1) * stride + e];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (r0 + j < ranges) v += u[j];
+        }
+        dot = fmaf(v, other, dot);
+        *to = f32_to_bf16(fmaf(s, v, old));
+    }
+    if (!dots) return;
+    __shared__ float wsum[4];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) dot += __shfl_xor(dot, o, 64);
+    if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = dot;
+    __syncthreads();
+    if (threadIdx.x == 0) dots[blockIdx.x] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+}
+
 // dx, dcoef (fp32 or bf16) and d_scale_bias: each NULL where it is not wanted.  With dx wanted, the gradient of the scale, <dy . R, x>,
 // comes out of the random-bias product that dx needs anyway.
 int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x, int64_t ldx,
@@ -494,6 +527,30 @@ int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, fl
         q = {(const float *)x, ldx, (d->tokens - 1) * ldx + d->in_f, nullptr, 0, 0, nullptr, 0, nullptr, d->tokens, d->out_f, d->in_f,
              0, 0, 0, 0, d->seed, (uint32_t)d->in_f, 1u};
         q.dotm = (const float *)dy, q.lddot = lddy;
+    }
+    // dx of bf16 layers in as many ranges of the output features as pay and as the workspace, whose t and partial matrices are used up, holds: few
+    // tokens are a handful of tiles otherwise, each with all of out_f to hash, split and multiply (us, with the sums: 502 x 527 -> 2918, k = 251: 87 -> 28;
+    // 942 x 729 -> 6529, k = 92: 179 -> 59; 1346 x 289 -> 5636, k = 48: 143 -> 38; 1494 x 2739 -> 8065, k = 105: 667 -> 396)
+    const int64_t stride = up256(q.M * q.N * 4) / 4, room = (reinterpret_cast<char *>(dots) - static_cast<char *>(workspace)) / (stride * 4);
+    const FgPlan rp = fg_plan(q.M, q.N, q.K, num_cus, dx && d->act_dtype == RDB_BF16 ? (int)std::max<int64_t>(1, std::min<int64_t>(room, 32)) : 1, true, FG_HOST_US);
+    if (rp.ranges > 1) {
+        FgProduct p = q;
+        p.a_es = fg_es(d->act_dtype);
+        p.bm = rp.bm;
+        p.groups = rp.groups;
+        p.out = static_cast<float *>(workspace);
+        p.ldo = q.N;
+        p.kchunk = fg_chunk(q.K, rp.ranges);
+        p.split_stride = stride;
+        p.dotm = nullptr;
+        if (int rc = fg_launch<FG_KCONT, FG_NOISE_1D>(p, num_cus, s, "f32_gemm_kernel (dy . R in ranges)")) return rc;
+        const int blocks = (int)std::min<int64_t>(cdiv(d->tokens, 64) * cdiv(std::max(d->in_f, d->out_f), FG_BN), cdiv(q.M * q.N, 256));   // of room for dots
+        f32_rbias_sum_kernel<<<blocks, 256, 0, s>>>(static_cast<bf16_t *>(dx), lddx, p.out, stride, rp.ranges, static_cast<const bf16_t *>(scale_bias),
+                                                    static_cast<const bf16_t *>(x), ldx, d_scale_bias ? dots : nullptr, (uint32_t)(q.M * q.N), (uint32_t)q.N);
+        if (int rc = check_launch("f32_rbias_sum_kernel")) return rc;
+        if (!d_scale_bias) return RDB_OK;
+        f32_sum_scalars_kernel<<<1, 256, 0, s>>>(d_scale_bias, dots, blocks);
+        return check_launch("f32_sum_scalars_kernel");
     }
     const FgPlan pl = fg_plan(q.M, q.N, q.K, num_cus, 1, true);
     q.bm = pl.bm;

@@ -1002,7 +1002,8 @@ template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_
     };
     if constexpr (BSRC == FG_NOISE_1D) {   // the random-bias products: added on top of an output, and / or reduced against a matrix
         if (q.scale) run(std::integral_constant<int, FG_ADD_SCALED>{});
-        else run(std::integral_constant<int, FG_DOT>{});
+        else if (q.dotm) run(std::integral_constant<int, FG_DOT>{});
+        else run(std::integral_constant<int, FG_STORE>{});   // a range's share, for f32_rbias_sum_kernel
     } else if (Groups::scaled && q.scale) {   // materialising W with its random-bias share
         if constexpr (Groups::scaled) {
             if (q.bm == 128) FG_LAUNCH(128, FG_STORE_RBIAS);

@@ -242,9 +242,10 @@ static int64_t z_behind(const rdb_linear_desc *d)
 {
     const int num_cus = num_compute_units();
     const int64_t zt = up256(d->tokens * d->k * 4), in_y = std::max<int64_t>(1, d->tokens * d->out_f * fg_es(d->act_dtype) / zt);
-    if (z_room(d, num_cus) < 3 * in_y) return 0;
+    const int most = z_room(d, num_cus);
+    if (most < 3 * in_y) return 0;
     // by the layer alone, whatever products are asked for (rdb_set_f32_split): what is kept may be larger than they need, never smaller
-    const int want = fg_plan(d->tokens, d->k, d->in_f, num_cus, std::max(1, z_room(d, num_cus)), FgGroups<FG_KCONT, FG_NOISE_M>::four, z_host_us(d), true).ranges;
+    const int want = fg_plan(d->tokens, d->k, d->in_f, num_cus, std::max(1, most), FgGroups<FG_KCONT, FG_NOISE_M>::four, z_host_us(d), true).ranges;
     return want >= 3 * in_y ? want * zt : 0;
 }
 // z into `z`, y (or NULL) to come, with what z_behind says behind z
@@ -592,6 +593,7 @@ static bool fg_state_ok(const rdb_linear_desc *d)
 {
     return d->act_dtype == RDB_F32 && d->coef_dtype == RDB_F32 && fg_ok(d) && d->tokens * std::max(d->in_f, d->out_f) < (1ll << 28);
 }
+bool linear_f32_state_ok(const rdb_linear_desc *d) { return fg_state_ok(d); }
 int64_t linear_f32_state_bytes(const rdb_linear_desc *d) { return fg_state_ok(d) ? 256 + up256(d->tokens * d->k * 4) + z_behind(d) : 0; }
 static float *fg_state_z(const void *state) { return reinterpret_cast<float *>(static_cast<char *>(const_cast<void *>(state)) + 256); }
 

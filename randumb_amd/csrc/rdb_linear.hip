@@ -321,6 +321,7 @@ bool f32_products_first(const rdb_linear_desc *d, bool dx);   // ahead of the fe
 int linear_dx_f32(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *coef, const void *scale_bias, const rdb_linear_desc *d,
                   int num_cus, void *workspace, int64_t workspace_bytes, hipStream_t s);
 int64_t linear_f32_state_bytes(const rdb_linear_desc *d);
+bool linear_f32_state_ok(const rdb_linear_desc *d);   // whether there is one: the bytes take a plan of the projection
 int64_t linear_f32_bwd_projected_workspace(const rdb_linear_desc *d, int num_cus);
 int64_t linear_dw_f32_workspace(const rdb_linear_desc *d, int num_cus);
 int linear_dw_f32(float *dW, const void *dy, int64_t lddy, const void *x, int64_t ldx, const rdb_linear_desc *d, int num_cus, hipStream_t s);
@@ -986,7 +987,7 @@ static int check_projected_f32(const char *who, const rdb_linear_desc *d)
 {
     int rc = check_desc(who, d);
     if (rc) return rc;
-    if (linear_f32_state_bytes(d) <= 0)
+    if (!linear_f32_state_ok(d))
         return set_error(RDB_E_UNSUPPORTED, "%s: the projected form in fp32 needs matrix-coef, fp32 activations and coefficients, non-empty sizes "
                                             "and tokens * max(in_f, out_f) below 2^28", who);
     return RDB_OK;
@@ -1002,7 +1003,8 @@ extern "C" int64_t rdb_linear_projection_bytes(const rdb_linear_desc *d)
 // What a training step should do with the layer: the rule behind the header's description, in integers.
 extern "C" int rdb_linear_projection_preferred(const rdb_linear_desc *d)
 {
-    if (!d || rdb_linear_projection_bytes(d) <= 0) return 0;
+    if (!d) return 0;
+    if (f32_projected(d) ? check_desc("rdb_linear_projection_preferred", d) || !linear_f32_state_ok(d) : rdb_linear_projection_bytes(d) <= 0) return 0;
     const int64_t k = d->k, in_f = d->in_f, out_f = d->out_f, T = d->tokens;
     const bool f32 = d->act_dtype == RDB_F32;
     // the few-token regimes, whose vector-ALU kernels have no projected form: the three one-call entry points take them
@@ -1047,7 +1049,7 @@ extern "C" int rdb_linear_projection_layout(const rdb_linear_desc *d, int64_t *i
 extern "C" int rdb_linear_projection_chunks(const rdb_linear_desc *d, int64_t *chunk_tokens)
 {
     if (f32_projected(d)) {
-        const bool ok = !check_desc("rdb_linear_projection_chunks", d) && linear_f32_state_bytes(d) > 0;
+        const bool ok = !check_desc("rdb_linear_projection_chunks", d) && linear_f32_state_ok(d);
         if (chunk_tokens) *chunk_tokens = ok ? d->tokens : 0;
         return ok ? 1 : 0;
     }

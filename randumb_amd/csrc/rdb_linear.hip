@@ -963,8 +963,9 @@ static ChunkPlan chunk_plan(const rdb_linear_desc *d)
     else per_chunk = d->tokens;
     pl.chunk_tokens = per_chunk;
     pl.nchunks = (int)cdiv(d->tokens, per_chunk);
-    const rdb_linear_desc first = chunk_desc(d, pl, 0);
-    pl.state_stride = linear_projection_bytes(&first);
+    // the last chunk, with fewer tokens, has fewer tiles and so may have more ranges of the projection, whose sums take more room
+    const rdb_linear_desc first = chunk_desc(d, pl, 0), last = chunk_desc(d, pl, pl.nchunks - 1);
+    pl.state_stride = std::max(linear_projection_bytes(&first), linear_projection_bytes(&last));
     if (pl.state_stride <= 0) pl.nchunks = 0;
     return pl;
 }

@@ -188,7 +188,8 @@ enum {
 enum { RDB_OP_LINEAR_FWD = 0, RDB_OP_LINEAR_BWD_DX = 1, RDB_OP_LINEAR_BWD_DCOEF = 2, RDB_OP_LINEAR_BWD_PROJECTED = 3,
        RDB_OP_LINEAR_BWD_PROJECTED_TO = 4, RDB_OP_LINEAR_BWD_DX_DSCALE = 5, RDB_OP_LINEAR_RBIAS_BWD = 6,
        RDB_OP_LINEAR_BWD_KEPT = 7, RDB_OP_LINEAR_RBIAS_FWD = 8,
-       RDB_OP_LINEAR_PROJECT_FWD_RBIAS = 9, RDB_OP_LINEAR_RBIAS_BWD_FULL = 10 };
+       RDB_OP_LINEAR_PROJECT_FWD_RBIAS = 9, RDB_OP_LINEAR_RBIAS_BWD_FULL = 10, RDB_OP_LINEAR_PROJECT = 11,
+       RDB_OP_LINEAR_FWD_KEPT = 12 };
 
 /* Device scratch (bytes) that entry point `op` can use for `desc`; 0 when it has no use for any.  A NULL or too small
  * workspace is never an error with RDB_ALGO_AUTO: the library then runs a kernel that needs none. */
@@ -330,6 +331,16 @@ int rdb_linear_projection_layout(const rdb_linear_desc *desc, int64_t *info);
 int rdb_linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *desc,
                        void *stream);
 
+/* rdb_linear_project and rdb_linear_project_fwd with scratch, rdb_linear_workspace_bytes(RDB_OP_LINEAR_PROJECT, desc) bytes, 16-byte
+ * aligned; 0 for most layers.  Where few tiles of z have long contractions, these run in ranges over the whole chip, and the ranges' sums lie in
+ * y's rows until y is written; layers with a y too narrow for that put them into the scratch, which is the call's own: nothing reads it
+ * afterwards.  Without it (NULL, or less) a tile's ranges run one after the other, in bf16 to the same bits (fp32: as many ranges as y holds). */
+int rdb_linear_project_ws(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *desc,
+                          void *workspace, int64_t workspace_bytes, void *stream);
+int rdb_linear_project_fwd_ws(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef,
+                              const void *bias, const rdb_linear_desc *desc, void *workspace, int64_t workspace_bytes,
+                              void *stream);
+
 /* rdb_linear_project (with coef) and rdb_linear_fwd_projected in one call: state <- projection of x and transposed coef,
  * y[t, o] = sum_m z[t, m] * coef[o, m] (+ bias[o]); coef must be bf16.  The forward pass of a training step (R.py:942-946
  * with what autograd saves replaced by the state).  With k <= 256 it is a single kernel launch: the blocks that multiply
@@ -372,7 +383,7 @@ int rdb_linear_bwd_projected_to(void *dx, int64_t lddx, void *dcoef, int dcoef_d
 
 /* The projected form's counterpart for layers without a projection state (bf16 with sizes that are not multiples of 8, fp32
  * in the few-token regime; rdb_linear_kept_bytes says how much, 0: none, use the calls above): the forward pass leaves
- * z = x . N^T (fp32, [tokens x k] row-major, and behind it scratch of the call's own) in `kept`, 16-byte aligned, and the backward pass starts from it.  scale_bias as
+ * z = x . N^T (fp32, [tokens x k] row-major) in `kept`, 16-byte aligned, and the backward pass starts from it.  scale_bias as
  * in rdb_linear_fwd.  rdb_linear_bwd_kept: dx, dcoef (dcoef_dtype RDB_F32 or RDB_BF16) and d_scale_bias (fp32) are
  * overwritten, NULL where not wanted; x is read for d_scale_bias only; a workspace of
  * rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_KEPT, desc) bytes.  Sums in a fixed order. */
@@ -383,6 +394,11 @@ int rdb_linear_fwd_kept(void *y, int64_t ldy, void *kept, const void *x, int64_t
  * floats, overwritten) are formed beside the projection, in the same launch.  RDB_E_UNSUPPORTED: another dtype, k or out_f of 2^31 or more. */
 int rdb_linear_fwd_kept_pseudo_bias(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef,
                                     const void *scale_bias, const rdb_pseudo_bias *bias, const rdb_linear_desc *desc, void *stream);
+/* Both (bias or pseudo_bias, or neither) with scratch for the projection as in rdb_linear_project_ws:
+ * rdb_linear_workspace_bytes(RDB_OP_LINEAR_FWD_KEPT, desc) bytes, 0 for most layers. */
+int rdb_linear_fwd_kept_ws(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef,
+                           const void *scale_bias, const void *bias, const rdb_pseudo_bias *pseudo_bias,
+                           const rdb_linear_desc *desc, void *workspace, int64_t workspace_bytes, void *stream);
 int rdb_linear_bwd_kept(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy,
                         int64_t lddy, const void *x, int64_t ldx, const void *kept, const void *coef,
                         const void *scale_bias, const rdb_linear_desc *desc, void *workspace, int64_t workspace_bytes,

@@ -18,6 +18,8 @@ RDB_OP_LINEAR_FWD, RDB_OP_LINEAR_BWD_DX, RDB_OP_LINEAR_BWD_DCOEF, RDB_OP_LINEAR_
 RDB_OP_LINEAR_BWD_DX_DSCALE = 5
 RDB_OP_LINEAR_RBIAS_BWD = 6
 RDB_OP_LINEAR_BWD_KEPT = 7
+RDB_OP_LINEAR_PROJECT = 11
+RDB_OP_LINEAR_FWD_KEPT = 12
 
 # every exported entry point, in header order; tests check the list against the built library
 EXPORTS = [
@@ -56,6 +58,8 @@ EXPORTS = [
     "rdb_linear_projection_layout",
     "rdb_linear_project",
     "rdb_linear_project_fwd",
+    "rdb_linear_project_ws",
+    "rdb_linear_project_fwd_ws",
     "rdb_linear_fwd_projected",
     "rdb_linear_bwd_dcoef_projected",
     "rdb_linear_bwd_projected",
@@ -64,6 +68,7 @@ EXPORTS = [
     "rdb_linear_kept_bytes",
     "rdb_linear_fwd_kept",
     "rdb_linear_fwd_kept_pseudo_bias",
+    "rdb_linear_fwd_kept_ws",
     "rdb_linear_bwd_kept",
     "rdb_set_big_tiles",
     "rdb_set_f32_split",
@@ -199,6 +204,10 @@ def load() -> ctypes.CDLL:
     L.rdb_linear_projection_layout.restype = ci
     L.rdb_linear_project.argtypes = [vp, vp, i64, vp, dp, vp]
     L.rdb_linear_project_fwd.argtypes = [vp, i64, vp, vp, i64, vp, vp, dp, vp]
+    L.rdb_linear_project_ws.argtypes = [vp, vp, i64, vp, dp, vp, i64, vp]
+    L.rdb_linear_project_ws.restype = ci
+    L.rdb_linear_project_fwd_ws.argtypes = [vp, i64, vp, vp, i64, vp, vp, dp, vp, i64, vp]
+    L.rdb_linear_project_fwd_ws.restype = ci
     L.rdb_linear_fwd_projected.argtypes = [vp, i64, vp, vp, vp, dp, vp]
     L.rdb_linear_bwd_dcoef_projected.argtypes = [vp, vp, i64, vp, dp, vp]
     L.rdb_linear_bwd_projected.argtypes = [vp, i64, vp, vp, i64, vp, vp, dp, vp, i64, vp]
@@ -210,6 +219,8 @@ def load() -> ctypes.CDLL:
     L.rdb_linear_fwd_kept.restype = ci
     L.rdb_linear_fwd_kept_pseudo_bias.argtypes = [vp, i64, vp, vp, i64, vp, vp, vp, dp, vp]
     L.rdb_linear_fwd_kept_pseudo_bias.restype = ci
+    L.rdb_linear_fwd_kept_ws.argtypes = [vp, i64, vp, vp, i64, vp, vp, vp, vp, dp, vp, i64, vp]
+    L.rdb_linear_fwd_kept_ws.restype = ci
     L.rdb_linear_bwd_kept.argtypes = [vp, i64, vp, ci, vp, vp, i64, vp, i64, vp, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_bwd_kept.restype = ci
     L.rdb_set_big_tiles.argtypes = [ci]

@@ -233,28 +233,29 @@ static int fg_project(float *z, const float *x, int64_t ldx, const rdb_linear_de
                                                   "f32_gemm_kernel (z = x . N^T)", z_host_us(d));
 }
 
-// Where the forward pass puts the partial matrices of z's ranges: into y, which is written last, or, where y holds less than a third of those that pay, behind
-// the z that is kept (32 MB at most: ranges times tiles are at most two to a compute unit, a tile 64 KB).  With the ranges that y holds instead,
+// Where the forward pass puts the partial matrices of z's ranges: into y, which is written last, or, where y holds less than a third of those that pay, into
+// scratch of the call's own (32 MB at most: ranges times tiles are at most two to a compute unit, a tile 64 KB), no part of what is kept.  With the ranges that y holds instead,
 // z of 492 tokens x 3184 -> 273, k = 118 in bf16, one range: 80 us, now 12.1 and 4 for the sums; 300 x 4000 -> 301, k = 100: 99, 9.2; 700 x 4000 -> 256, k =
-// 120 in fp32: 63, 13.9.  Where it holds more, what is kept does not grow for the 3 to 5 us
+// 120 in fp32: 63, 13.9.  Where it holds more, scratch is not asked for the 3 to 5 us
 // that are left (433 x 3320 -> 1288, k = 144: 18.3, 15.0; 128 x 784 -> 256, k = 64: four ranges, nine would pay).
-static int64_t z_behind(const rdb_linear_desc *d)
+static int64_t z_scratch(const rdb_linear_desc *d)
 {
     const int num_cus = num_compute_units();
     const int64_t zt = up256(d->tokens * d->k * 4), in_y = std::max<int64_t>(1, d->tokens * d->out_f * fg_es(d->act_dtype) / zt);
     const int most = z_room(d, num_cus);
     if (most < 3 * in_y) return 0;
-    // by the layer alone, whatever products are asked for (rdb_set_f32_split): what is kept may be larger than they need, never smaller
+    // by the layer alone, whatever products are asked for (rdb_set_f32_split): it may be larger than they need, never smaller
     const int want = fg_plan(d->tokens, d->k, d->in_f, num_cus, std::max(1, most), FgGroups<FG_KCONT, FG_NOISE_M>::four, z_host_us(d), true).ranges;
     return want >= 3 * in_y ? want * zt : 0;
 }
-// z into `z`, y (or NULL) to come, with what z_behind says behind z
-static int fg_project_kept(float *z, const void *x, int64_t ldx, void *y, int64_t ldy, const rdb_linear_desc *d, int num_cus, hipStream_t s, const FgValues &values)
+// z into `z`, y (or NULL) to come; scratch: NULL, or scratch_bytes (less than z_scratch, or not aligned: y's room, as without)
+static int fg_project_kept(float *z, const void *x, int64_t ldx, void *y, int64_t ldy, const rdb_linear_desc *d, int num_cus, void *scratch, int64_t scratch_bytes,
+                           hipStream_t s, const FgValues &values)
 {
-    const int64_t zt = up256(d->tokens * d->k * 4), behind = z_behind(d);
+    const int64_t zt = up256(d->tokens * d->k * 4), asked = scratch && fg_aligned16(scratch) ? z_scratch(d) : 0;
     float *part = z;
     int64_t room = 0;
-    if (behind) part = z + zt / 4, room = behind;
+    if (asked > 0 && scratch_bytes >= asked) part = static_cast<float *>(scratch), room = asked;
     else if (y && ldy == d->out_f && fg_aligned16(y)) part = static_cast<float *>(y), room = d->tokens * d->out_f * fg_es(d->act_dtype);
     return fg_project(z, static_cast<const float *>(x), ldx, d, num_cus, s, part, (int)std::min<int64_t>(32, room / zt), values);
 }
@@ -413,7 +414,7 @@ bool f32_products_first(const rdb_linear_desc *d, bool dx)
 // in fp32 below 32 and where the vector-ALU kernels' three calls take less: their coefficient gradient projects x again, 5 us more
 // than their forward pass, against 10 here) stay with the kernels of rdb_smallk.hip.  4097 tokens x 1001 -> 999, k = 100 in bf16, forward and backward:
 // 122 -> 98 us; 128 tokens x 784 -> 256, k = 64 in fp32: 22.7 + 11.1 + 27.8 us of few-token kernels -> 17 + 6.
-int64_t linear_kept_f32_z_bytes(const rdb_linear_desc *d)
+int64_t linear_kept_f32_bytes(const rdb_linear_desc *d)
 {
     if (!fg_ok(d) || d->algo != RDB_ALGO_AUTO || d->tokens * std::max(d->in_f, d->out_f) >= (1ll << 28) || d->sO != d->in_f || d->sI != 1) return 0;
     const bool b16 = d->act_dtype == RDB_BF16;
@@ -421,11 +422,7 @@ int64_t linear_kept_f32_z_bytes(const rdb_linear_desc *d)
     if (!b16 && d->k <= 64 && f32_products_us(d, false) + f32_products_us(d, true) + 10.0 > 3.0 * few_token_us(d) + 5.0) return 0;
     return up256(d->tokens * d->k * 4);
 }
-int64_t linear_kept_f32_bytes(const rdb_linear_desc *d)
-{
-    const int64_t z = linear_kept_f32_z_bytes(d);
-    return z ? z + z_behind(d) : 0;
-}
+int64_t linear_kept_f32_scratch(const rdb_linear_desc *d) { return linear_kept_f32_bytes(d) ? z_scratch(d) : 0; }
 
 static int fg_rbias(FgProduct q, const void *scale, const rdb_linear_desc *d, int num_cus, hipStream_t s, const char *name)
 {
@@ -438,16 +435,16 @@ static int fg_rbias(FgProduct q, const void *scale, const rdb_linear_desc *d, in
 
 // values: NULL, or a pseudorandom bias whose values the launch of the projection forms on the side (an fp32 layer's; then `bias`)
 int linear_fwd_kept_f32(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
-                        const rdb_pseudo_bias *values, const rdb_linear_desc *d, int num_cus, hipStream_t s)
+                        const rdb_pseudo_bias *values, const rdb_linear_desc *d, int num_cus, void *scratch, int64_t scratch_bytes, hipStream_t s)
 {
     FgValues v = {};
     if (values) {
         v = {values->values, values->coef, values->scale, (int)d->out_f, (int)values->k, values->seed};
         bias = values->values;
     }
-    if (!linear_kept_f32_z_bytes(d) || !fg_aligned16(kept) || d->tokens * ldx >= (1ll << 29) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
+    if (!linear_kept_f32_bytes(d) || !fg_aligned16(kept) || d->tokens * ldx >= (1ll << 29) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     float *z = static_cast<float *>(kept);
-    if (int rc = fg_project_kept(z, x, ldx, y, ldy, d, num_cus, s, v)) return rc;
+    if (int rc = fg_project_kept(z, x, ldx, y, ldy, d, num_cus, scratch, scratch_bytes, s, v)) return rc;
     FgProduct q = {z, d->k, d->tokens * d->k, (const float *)coef, d->k, d->out_f * d->k, (float *)y, ldy, (const float *)bias, d->tokens, d->out_f, d->k,
                    0, 0, 0, 0, d->seed};
     q.b_es = fg_es(d->coef_dtype);
@@ -463,7 +460,7 @@ int linear_fwd_kept_f32(void *y, int64_t ldy, void *kept, const void *x, int64_t
 // [tokens x out_f])
 int64_t linear_bwd_kept_f32_workspace(const rdb_linear_desc *d, int num_cus)
 {
-    if (!linear_kept_f32_z_bytes(d)) return 0;
+    if (!linear_kept_f32_bytes(d)) return 0;
     const int r = dc_room(d, num_cus);
     return linear_f32_workspace(RDB_OP_LINEAR_BWD_DX, d, num_cus) + (r > 1 ? (int64_t)r * up256(d->out_f * d->k * 4) : 0) +
            up256(cdiv(d->tokens, 64) * cdiv(std::max(d->in_f, d->out_f), FG_BN) * 4);
@@ -508,7 +505,7 @@ int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, fl
                         const void *kept, const void *coef, const void *scale_bias, const rdb_linear_desc *d, int num_cus, void *workspace,
                         int64_t workspace_bytes, hipStream_t s)
 {
-    if (!linear_kept_f32_z_bytes(d) || !fg_aligned16(kept) || !workspace || !fg_aligned16(workspace) ||
+    if (!linear_kept_f32_bytes(d) || !fg_aligned16(kept) || !workspace || !fg_aligned16(workspace) ||
         workspace_bytes < linear_bwd_kept_f32_workspace(d, num_cus) || d->tokens * lddy >= (1ll << 29) || (dx && d->tokens * lddx >= (1ll << 29)) ||
         (d_scale_bias && d->tokens * ldx >= (1ll << 29)))
         return RDB_E_UNSUPPORTED;
@@ -593,8 +590,8 @@ static bool fg_state_ok(const rdb_linear_desc *d)
 {
     return d->act_dtype == RDB_F32 && d->coef_dtype == RDB_F32 && fg_ok(d) && d->tokens * std::max(d->in_f, d->out_f) < (1ll << 28);
 }
-bool linear_f32_state_ok(const rdb_linear_desc *d) { return fg_state_ok(d); }
-int64_t linear_f32_state_bytes(const rdb_linear_desc *d) { return fg_state_ok(d) ? 256 + up256(d->tokens * d->k * 4) + z_behind(d) : 0; }
+int64_t linear_f32_state_bytes(const rdb_linear_desc *d) { return fg_state_ok(d) ? 256 + up256(d->tokens * d->k * 4) : 0; }
+int64_t linear_project_f32_scratch(const rdb_linear_desc *d) { return fg_state_ok(d) ? z_scratch(d) : 0; }
 static float *fg_state_z(const void *state) { return reinterpret_cast<float *>(static_cast<char *>(const_cast<void *>(state)) + 256); }
 
 // workspace of the backward pass from the state: t = dy . C with the partial matrices of its ranges, then the partial matrices
@@ -614,14 +611,14 @@ static int fg_fwd_from_z(void *y, int64_t ldy, const float *z, const void *coef,
 }
 
 // state <- z.  The partial matrices of the projection's contraction ranges lie in y's memory, which is written last (only when y is
-// contiguous, and as many ranges as fit there; without y the contraction runs in one range), or behind z where y is too narrow for them.
+// contiguous, and as many ranges as fit there; without y the contraction runs in one range), or in scratch where y is too narrow for them.
 int linear_project_f32(void *state, void *y, int64_t ldy, const void *x, int64_t ldx, const void *coef, const void *bias, const rdb_linear_desc *d,
-                       int num_cus, hipStream_t s)
+                       int num_cus, void *scratch, int64_t scratch_bytes, hipStream_t s)
 {
     if (!fg_state_ok(d) || !fg_aligned16(state) || d->tokens * ldx >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     if (y && (d->tokens * ldy >= (1ll << 29))) return RDB_E_UNSUPPORTED;
     float *z = fg_state_z(state);
-    if (int rc = fg_project_kept(z, x, ldx, y, ldy, d, num_cus, s, {})) return rc;
+    if (int rc = fg_project_kept(z, x, ldx, y, ldy, d, num_cus, scratch, scratch_bytes, s, {})) return rc;
     if (!y) return RDB_OK;
     return fg_fwd_from_z(y, ldy, z, coef, bias, d, num_cus, s);
 }

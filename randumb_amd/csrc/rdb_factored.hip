@@ -46,7 +46,7 @@ struct ZParams {
     // part == NULL: every block runs its tile's ranges one after the other.  Otherwise the grid holds a block per tile and range,
     // range by range; the blocks of the last range of a tile wait for the others' sums.  A token tile's sums lie in its tokens' rows, of
     // part_row bytes each, of y, which nobody writes before they have been read (a multiplying block waits for all of its tokens' z),
-    // or behind the state: [coefficient tile][range][token of the tile][32] floats, and behind them, at the end of the rows, a tag for each.
+    // or in the call's own scratch: [coefficient tile][range][token of the tile][32] floats, and behind them, at the end of the rows, a tag for each.
     int ranges, range_stages;
     char *part;
     int64_t part_row;
@@ -455,8 +455,8 @@ int linear_fwd_projected(void *y, int64_t ldy, const void *state, const void *co
 // tiles than compute units the others stand idle meanwhile (2000 tokens x 4096 features, k = 256: 64 tiles of 64 stages).  So as
 // many ranges as leave a unit for every block, of at least KZ_MIN_STAGES stages: below that the wait for the others' sums and
 // fetching them (some 4 us) costs what the shorter loop saves.  The numbers depend on the layer alone, so that the same sums in the same
-// order come out wherever they are computed.  The sums need (ranges - 1) * kpad * 4 bytes of a token's out_f * 2 in y; layers too narrow for that have
-// room behind their state, 9 MB at most (ranges times tiles are at most the compute units, a sum 32 KB).  With as many ranges as y holds instead: 640
+// order come out wherever they are computed.  The sums need (ranges - 1) * kpad * 4 bytes of a token's out_f * 2 in y; layers too narrow for that take
+// scratch of the call's own, 9 MB at most (ranges times tiles are at most the compute units, a sum 32 KB).  With as many ranges as y holds instead: 640
 // tokens x 3400 -> 696, k = 264, one range: 28.6 us, now 20.4; 200 x 8000 -> 1000, k = 400: 39.2, 24.2; 700 x 4000 -> 400, k = 200: 42.6, 26.4; 1056 x
 // 3072 -> 768, k = 240, two ranges: 28.6, 25.5; 2048 x 3072 -> 768, k = 256: 27.8, 24.8.
 constexpr int KZ_MIN_STAGES = 8, KZ_MAX_RANGES = 16;
@@ -475,8 +475,9 @@ static int64_t z_part_row(const rdb_linear_desc *d, int ranges)
     const int64_t kpad = cdiv(d->k, 64) * 64, row = (ranges - 1) * (kpad * 4 + kpad / 4);
     return row + 64 > d->out_f * 2 ? row : 0;
 }
-// the state, and behind it room for the ranges' sums of layers whose y has none, which a transient state may do without
-int64_t linear_projection_extra(const rdb_linear_desc *d)
+// Scratch for the ranges' sums of layers whose y has no room for them.  Used by the projecting launch alone: it is no part of the state that is kept for
+// the backward pass (2048 tokens x 3072 -> 768, k = 256: a state of 2.5 MB, scratch of 6.7).  Without it a tile's block adds its ranges up itself.
+int64_t linear_projection_scratch(const rdb_linear_desc *d)
 {
     const ProjLayout L = proj_layout(d);
     if (!L.ok) return 0;
@@ -484,7 +485,12 @@ int64_t linear_projection_extra(const rdb_linear_desc *d)
     z_ranges(d, (int)(L.kpad / KZ_BM * cdiv(d->tokens, KZ_BT)), ranges, range_stages);
     return ranges > 1 ? (d->tokens * z_part_row(d, ranges) + 255) / 256 * 256 : 0;
 }
-int64_t linear_projection_bytes(const rdb_linear_desc *d) { return proj_layout(d).bytes + linear_projection_extra(d); }
+int64_t linear_projection_bytes(const rdb_linear_desc *d) { return proj_layout(d).bytes; }
+// `scratch` if it is such scratch
+static void *enough_scratch(void *scratch, int64_t bytes, const rdb_linear_desc *d)
+{
+    return scratch && aligned16(scratch) && bytes > 0 && bytes >= linear_projection_scratch(d) ? scratch : nullptr;
+}
 
 static bool fill_z_params(ZParams &p, void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d)
 {
@@ -519,14 +525,14 @@ static bool fill_z_params(ZParams &p, void *state, const void *x, int64_t ldx, c
 }
 
 // Spreads the ranges of a split contraction over blocks of their own, with the sums on the way in y's rows (contiguous, not yet
-// written) or, where those are too short, behind the state (room: it has its extra bytes).  False when there is nothing to spread, or no place.
-static bool spread_ranges(ZParams &p, void *state, void *y, int64_t ldy, const rdb_linear_desc *d, bool room, int *rc)
+// written) or, where those are too short, in `scratch` (NULL, or linear_projection_scratch bytes).  False when there is nothing to spread, or no place.
+static bool spread_ranges(ZParams &p, void *state, void *y, int64_t ldy, const rdb_linear_desc *d, void *scratch, int *rc)
 {
     *rc = RDB_OK;
     if (p.ranges <= 1 || !one_launch_mode()) return false;
     if (const int64_t row = z_part_row(d, p.ranges)) {
-        if (!room) return false;
-        p.part = static_cast<char *>(state) + proj_layout(d).bytes;
+        if (!scratch) return false;
+        p.part = static_cast<char *>(scratch);
         p.part_row = row;
         p.part_stays = 1;
     } else if (y && ldy == d->out_f && aligned16(y)) {
@@ -556,12 +562,12 @@ static void set_z_grid(ZParams &p, int z_grid, int num_cus)
 static size_t z_smem() { return engine_smem<KZ_BM, KZ_BT, F_BK, K_CONT, K_CONT>(); }
 
 // y: NULL, or the rows of the forward product to come, free to hold sums on the way
-static int launch_z(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, bool room, hipStream_t s)
+static int launch_z(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, void *scratch, hipStream_t s)
 {
     ZParams p;
     int rc;
     if (!fill_z_params(p, state, x, ldx, coef, d)) return RDB_E_UNSUPPORTED;
-    const bool spread = spread_ranges(p, state, y, ldy, d, room, &rc);
+    const bool spread = spread_ranges(p, state, y, ldy, d, scratch, &rc);
     if (rc) return rc;
     const size_t smem = z_smem();
     const void *fn = p.ranges > 1 ? (const void *)factored_z_kernel<true> : (const void *)factored_z_kernel<false>;
@@ -573,21 +579,22 @@ static int launch_z(void *state, const void *x, int64_t ldx, const void *coef, v
     return check_launch("factored_z_kernel");
 }
 
-int linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, hipStream_t s, bool room)
+// scratch: NULL, or scratch_bytes; what is less than linear_projection_scratch, or not aligned, goes unused
+int linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, hipStream_t s, void *scratch, int64_t scratch_bytes)
 {
-    return launch_z(state, x, ldx, coef, nullptr, 0, d, room, s);
+    return launch_z(state, x, ldx, coef, nullptr, 0, d, enough_scratch(scratch, scratch_bytes, d), s);
 }
 
 // The same ahead of a forward product: y's rows, contiguous and written last, hold N or sums on the way meanwhile.  With a contraction in
 // several ranges the 256-wide tiles' sums would differ from launch_z's (z_ranges).
 int linear_project_before(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, int num_cus,
-                          hipStream_t s, bool state_room)
+                          hipStream_t s, void *scratch, int64_t scratch_bytes)
 {
     ZParams p;
     if (!fill_z_params(p, state, x, ldx, coef, d)) return RDB_E_UNSUPPORTED;
     const int64_t room = ldy == d->out_f && p.ranges == 1 ? d->tokens * d->out_f * (int64_t)sizeof(bf16_t) : 0;
     const int rc = linear_z_big(state, x, ldx, coef, y, room, d, num_cus, s);
-    return rc != RDB_E_UNSUPPORTED ? rc : launch_z(state, x, ldx, coef, y, ldy, d, state_room, s);
+    return rc != RDB_E_UNSUPPORTED ? rc : launch_z(state, x, ldx, coef, y, ldy, d, enough_scratch(scratch, scratch_bytes, d), s);
 }
 
 // The forward product's parameters when the contraction of a token fits in registers (z in fragment order); returns the
@@ -630,7 +637,7 @@ template <bool BIAS> static int launch_ys(const StParams &q, int items, hipStrea
 // contraction of a token fits in registers (k <= 256), otherwise in two.
 // polls: how long its multiplying blocks wait; fewer than SYNC_SPIN_LIMIT in a self-test only.
 int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, bool with_ct, const void *bias,
-                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls, bool room)
+                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls, void *scratch, int64_t scratch_bytes)
 {
     ZYParams p;
     if (!fill_z_params(p.z, state, x, ldx, with_ct ? coef : nullptr, d)) return RDB_E_UNSUPPORTED;
@@ -639,7 +646,7 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
         // check the second call's conditions before the first launch, so that a refusal leaves nothing half done
         if (d->coef_dtype != RDB_BF16 || ldy % 8 || !aligned16(y) || !aligned16(coef)) return RDB_E_UNSUPPORTED;
         if (((uintptr_t)bias & 7) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
-        if (int rc = linear_project_before(state, x, ldx, with_ct ? coef : nullptr, y, ldy, d, num_cus, s, room)) return rc;
+        if (int rc = linear_project_before(state, x, ldx, with_ct ? coef : nullptr, y, ldy, d, num_cus, s, scratch, scratch_bytes)) return rc;
         return linear_fwd_projected(y, ldy, state, coef, bias, d, num_cus, s);
     }
     const ProjLayout L = proj_layout(d);
@@ -652,7 +659,7 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
     p.y.sync_wait.polls = polls;
     if (int rc = sync_giveups_ptr(&p.y.sync_wait.giveups)) return rc;
     int rc;
-    const bool spread = spread_ranges(p.z, state, y, ldy, d, room, &rc);
+    const bool spread = spread_ranges(p.z, state, y, ldy, d, enough_scratch(scratch, scratch_bytes, d), &rc);
     if (rc) return rc;
     set_z_grid(p.z, xcd_grid_size(p.z.tiles_m * p.z.tiles_t) * (spread ? p.z.ranges : 1), num_cus);
     return bias ? launch_zy<true>(p, y_items, s) : launch_zy<false>(p, y_items, s);
@@ -720,13 +727,15 @@ int linear_fwd_factored(void *y, int64_t ldy, const void *x, int64_t ldx, const 
                         const rdb_linear_desc *d, int num_cus, void *workspace, int64_t workspace_bytes, hipStream_t s)
 {
     if (scale_bias || d->coef_dtype != RDB_BF16 || !factored_shape_ok(d)) return RDB_E_UNSUPPORTED;  // the random-bias term is not low rank
-    if (!workspace || workspace_bytes < proj_layout(d).bytes) return RDB_E_UNSUPPORTED;
+    if (!workspace || workspace_bytes < linear_projection_bytes(d)) return RDB_E_UNSUPPORTED;
     if (d->algo == RDB_ALGO_AUTO && !cheaper_factored(d)) return RDB_E_UNSUPPORTED;
     // check everything before the first launch, so that a refusal leaves nothing half done
     if (d->tokens * ldx >= (1ll << 29) || ldx % 8 || ldy % 8 || !aligned16(x) || !aligned16(coef) || !aligned16(y) || !aligned16(workspace))
         return RDB_E_UNSUPPORTED;
     if (((uintptr_t)bias & 7) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
-    return linear_project_fwd(y, ldy, workspace, x, ldx, coef, false, bias, d, num_cus, s, SYNC_SPIN_LIMIT, workspace_bytes >= linear_projection_bytes(d));
+    const int64_t state = linear_projection_bytes(d);   // a multiple of 256; the scratch lies behind it
+    return linear_project_fwd(y, ldy, workspace, x, ldx, coef, false, bias, d, num_cus, s, SYNC_SPIN_LIMIT, static_cast<char *>(workspace) + state,
+                              workspace_bytes - state);
 }
 
 // dC = dy^T . (x . N^T) with the projection state in the workspace; dcoef must have been zeroed on the same stream.
@@ -734,12 +743,13 @@ int linear_dcoef_factored(float *dcoef, const void *dy, int64_t lddy, const void
                           void *workspace, int64_t workspace_bytes, hipStream_t s)
 {
     if (!factored_shape_ok(d)) return RDB_E_UNSUPPORTED;
-    if (!workspace || workspace_bytes < proj_layout(d).bytes) return RDB_E_UNSUPPORTED;
+    if (!workspace || workspace_bytes < linear_projection_bytes(d)) return RDB_E_UNSUPPORTED;
     if (d->algo == RDB_ALGO_AUTO && !cheaper_factored(d)) return RDB_E_UNSUPPORTED;
     if (d->tokens * ldx >= (1ll << 29) || d->tokens * lddy >= (1ll << 29) || ldx % 8 || lddy % 8 || !aligned16(x) || !aligned16(dy) ||
         !aligned16(workspace))
         return RDB_E_UNSUPPORTED;
-    int rc = linear_project(workspace, x, ldx, nullptr, d, s, workspace_bytes >= linear_projection_bytes(d));
+    const int64_t state = linear_projection_bytes(d);
+    int rc = linear_project(workspace, x, ldx, nullptr, d, s, static_cast<char *>(workspace) + state, workspace_bytes - state);
     if (rc) return rc;
     return linear_dcoef_projected(dcoef, dy, lddy, workspace, d, num_cus, s);
 }

@@ -285,10 +285,11 @@ int linear_fwd_strip(void *y, int64_t ldy, const void *x, int64_t ldx, const voi
 
 // rdb_factored.hip
 int64_t linear_projection_bytes(const rdb_linear_desc *d);
-int64_t linear_projection_extra(const rdb_linear_desc *d);
-int linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, hipStream_t s, bool room = true);
+int64_t linear_projection_scratch(const rdb_linear_desc *d);
+int linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, hipStream_t s, void *scratch = nullptr,
+                   int64_t scratch_bytes = 0);
 int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, bool with_ct, const void *bias,
-                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls = SYNC_SPIN_LIMIT, bool room = true);
+                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls = SYNC_SPIN_LIMIT, void *scratch = nullptr, int64_t scratch_bytes = 0);
 int linear_fwd_projected(void *y, int64_t ldy, const void *z, const void *coef, const void *bias, const rdb_linear_desc *d, int num_cus,
                          hipStream_t s);
 int linear_dcoef_projected(float *dcoef, const void *dy, int64_t lddy, const void *z, const rdb_linear_desc *d, int num_cus, hipStream_t s);
@@ -320,13 +321,13 @@ int linear_fwd_f32(void *y, int64_t ldy, const void *x, int64_t ldx, const void 
 bool f32_products_first(const rdb_linear_desc *d, bool dx);   // ahead of the few-token kernels
 int linear_dx_f32(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *coef, const void *scale_bias, const rdb_linear_desc *d,
                   int num_cus, void *workspace, int64_t workspace_bytes, hipStream_t s);
-int64_t linear_f32_state_bytes(const rdb_linear_desc *d);
-bool linear_f32_state_ok(const rdb_linear_desc *d);   // whether there is one: the bytes take a plan of the projection
+int64_t linear_f32_state_bytes(const rdb_linear_desc *d);   // 0: none
+int64_t linear_project_f32_scratch(const rdb_linear_desc *d);
 int64_t linear_f32_bwd_projected_workspace(const rdb_linear_desc *d, int num_cus);
 int64_t linear_dw_f32_workspace(const rdb_linear_desc *d, int num_cus);
 int linear_dw_f32(float *dW, const void *dy, int64_t lddy, const void *x, int64_t ldx, const rdb_linear_desc *d, int num_cus, hipStream_t s);
 int linear_project_f32(void *state, void *y, int64_t ldy, const void *x, int64_t ldx, const void *coef, const void *bias, const rdb_linear_desc *d,
-                       int num_cus, hipStream_t s);
+                       int num_cus, void *scratch, int64_t scratch_bytes, hipStream_t s);
 int linear_fwd_projected_f32(void *y, int64_t ldy, const void *state, const void *coef, const void *bias, const rdb_linear_desc *d, int num_cus,
                              hipStream_t s);
 int linear_bwd_projected_f32(void *dx, int64_t lddx, float *dcoef, const void *dy, int64_t lddy, const void *state, const void *coef,
@@ -364,7 +365,7 @@ int linear_dx_rbias_add_dscale(void *dx, int64_t lddx, void *dscale, int dscale_
 int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);
 int64_t rbias_scratch_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);   // rdb_rbias.hip
 int linear_project_before(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, int num_cus,
-                          hipStream_t s, bool state_room = true);   // rdb_factored.hip
+                          hipStream_t s, void *scratch, int64_t scratch_bytes);   // rdb_factored.hip
 int linear_fwd_rbias_big(void *y, int64_t ldy, const void *x, int64_t ldx, const void *state, const void *coef, const void *scale, const void *bias,
                          const rdb_linear_desc *d, void *table, int num_cus, hipStream_t s);
 
@@ -413,7 +414,8 @@ using namespace rdb;
 
 static int64_t bwd_projected_workspace(const rdb_linear_desc *d, bool force_partial);
 static int64_t bwd_projected_extra(const rdb_linear_desc *d);
-static int64_t project_fwd_rbias_table(const rdb_linear_desc *d);
+static int64_t project_fwd_rbias_bytes(const rdb_linear_desc *d);
+static int64_t project_scratch(const rdb_linear_desc *d);
 
 // vector-coef coefficient gradient in two passes: dW = dy^T . x into the workspace (and the partial matrices of its token
 // ranges), then the contraction of rdb_materialize_bwd and, for the scale's gradient, of rdb_scale_bias_bwd, with their scratch
@@ -434,7 +436,7 @@ static int64_t vec_dcoef_workspace(const rdb_linear_desc *d)
 
 static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d);
 namespace rdb {
-int64_t linear_kept_f32_z_bytes(const rdb_linear_desc *d);   // rdb_f32.hip
+int64_t linear_kept_f32_scratch(const rdb_linear_desc *d);   // rdb_f32.hip
 int64_t linear_bwd_kept_f32_workspace(const rdb_linear_desc *d, int num_cus);   // rdb_f32.hip
 }
 
@@ -442,6 +444,8 @@ static bool kept_layer(const rdb_linear_desc *d);
 extern "C" int64_t rdb_linear_workspace_bytes(int op, const rdb_linear_desc *d)
 {
     if (!d) return 0;
+    if (op == RDB_OP_LINEAR_PROJECT) return project_scratch(d);
+    if (op == RDB_OP_LINEAR_FWD_KEPT) return kept_layer(d) ? linear_kept_f32_scratch(d) : 0;
     if (op == RDB_OP_LINEAR_BWD_KEPT) return kept_layer(d) ? linear_bwd_kept_f32_workspace(d, num_compute_units()) : 0;
     int64_t need = linear_workspace_bytes_main(op, d);
     if (d->algo == RDB_ALGO_AUTO && d->act_dtype == RDB_BF16 && d->coef_rows != 0 &&
@@ -492,15 +496,15 @@ static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d)
         const int64_t more = op == RDB_OP_LINEAR_RBIAS_BWD_FULL ? rbias_scratch_bytes(d, d->in_f, num_compute_units()) : 0;
         return more > 0 ? rbias_dot_room(d) + more : linear_dx_rbias_dot_floats(d) * 4;   // ... and behind them R, or sums of ranges
     }
-    if (op == RDB_OP_LINEAR_PROJECT_FWD_RBIAS) return project_fwd_rbias_table(d);
+    if (op == RDB_OP_LINEAR_PROJECT_FWD_RBIAS) return project_fwd_rbias_bytes(d);
     if (op == RDB_OP_LINEAR_RBIAS_FWD)
         return d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16 ? rbias_scratch_bytes(d, d->out_f, num_compute_units()) : 0;
     if (op == RDB_OP_LINEAR_BWD_PROJECTED || op == RDB_OP_LINEAR_BWD_PROJECTED_TO) {
         const int64_t base = bwd_projected_workspace(d, op == RDB_OP_LINEAR_BWD_PROJECTED_TO), extra = base > 0 ? bwd_projected_extra(d) : 0;
         return extra > 0 ? (base + 255) / 256 * 256 + extra : base;   // what lies behind `base` is never required
     }
-    if (op == RDB_OP_LINEAR_FWD) return d->coef_dtype == RDB_BF16 ? linear_projection_bytes(d) : 0;
-    if (op == RDB_OP_LINEAR_BWD_DCOEF) return linear_projection_bytes(d);  // reads no coefficients: their dtype does not matter
+    if (op == RDB_OP_LINEAR_FWD) return d->coef_dtype == RDB_BF16 ? linear_projection_bytes(d) + linear_projection_scratch(d) : 0;
+    if (op == RDB_OP_LINEAR_BWD_DCOEF) return linear_projection_bytes(d) + linear_projection_scratch(d);  // reads no coefficients: their dtype does not matter
     return 0;
 }
 
@@ -919,7 +923,7 @@ extern "C" int rdb_linear_fwd_static(void *y, int64_t ldy, const void *x, int64_
     int rc = check_desc("rdb_linear_fwd_static", d);
     if (rc) return rc;
     int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_FWD, d);
-    if (need > RDB_STATIC_SCRATCH_BYTES && need == linear_projection_bytes(d)) need -= linear_projection_extra(d);   // goes without
+    if (need > RDB_STATIC_SCRATCH_BYTES && need == linear_projection_bytes(d) + linear_projection_scratch(d)) need = linear_projection_bytes(d);   // goes without
     if (need > RDB_STATIC_SCRATCH_BYTES)
         return set_error(RDB_E_WORKSPACE, "rdb_linear_fwd_static: this layer's kernels use %lld bytes of scratch, the library's static scratch holds "
                                           "%lld: call rdb_linear_fwd with a workspace of the caller's", (long long)need, (long long)RDB_STATIC_SCRATCH_BYTES);
@@ -963,9 +967,8 @@ static ChunkPlan chunk_plan(const rdb_linear_desc *d)
     else per_chunk = d->tokens;
     pl.chunk_tokens = per_chunk;
     pl.nchunks = (int)cdiv(d->tokens, per_chunk);
-    // the last chunk, with fewer tokens, has fewer tiles and so may have more ranges of the projection, whose sums take more room
-    const rdb_linear_desc first = chunk_desc(d, pl, 0), last = chunk_desc(d, pl, pl.nchunks - 1);
-    pl.state_stride = std::max(linear_projection_bytes(&first), linear_projection_bytes(&last));
+    const rdb_linear_desc first = chunk_desc(d, pl, 0);
+    pl.state_stride = linear_projection_bytes(&first);   // a state of fewer tokens is no larger
     if (pl.state_stride <= 0) pl.nchunks = 0;
     return pl;
 }
@@ -988,7 +991,7 @@ static int check_projected_f32(const char *who, const rdb_linear_desc *d)
 {
     int rc = check_desc(who, d);
     if (rc) return rc;
-    if (!linear_f32_state_ok(d))
+    if (linear_f32_state_bytes(d) <= 0)
         return set_error(RDB_E_UNSUPPORTED, "%s: the projected form in fp32 needs matrix-coef, fp32 activations and coefficients, non-empty sizes "
                                             "and tokens * max(in_f, out_f) below 2^28", who);
     return RDB_OK;
@@ -1004,8 +1007,7 @@ extern "C" int64_t rdb_linear_projection_bytes(const rdb_linear_desc *d)
 // What a training step should do with the layer: the rule behind the header's description, in integers.
 extern "C" int rdb_linear_projection_preferred(const rdb_linear_desc *d)
 {
-    if (!d) return 0;
-    if (f32_projected(d) ? check_desc("rdb_linear_projection_preferred", d) || !linear_f32_state_ok(d) : rdb_linear_projection_bytes(d) <= 0) return 0;
+    if (!d || rdb_linear_projection_bytes(d) <= 0) return 0;
     const int64_t k = d->k, in_f = d->in_f, out_f = d->out_f, T = d->tokens;
     const bool f32 = d->act_dtype == RDB_F32;
     // the few-token regimes, whose vector-ALU kernels have no projected form: the three one-call entry points take them
@@ -1050,7 +1052,7 @@ extern "C" int rdb_linear_projection_layout(const rdb_linear_desc *d, int64_t *i
 extern "C" int rdb_linear_projection_chunks(const rdb_linear_desc *d, int64_t *chunk_tokens)
 {
     if (f32_projected(d)) {
-        const bool ok = !check_desc("rdb_linear_projection_chunks", d) && linear_f32_state_ok(d);
+        const bool ok = !check_desc("rdb_linear_projection_chunks", d) && linear_f32_state_bytes(d) > 0;
         if (chunk_tokens) *chunk_tokens = ok ? d->tokens : 0;
         return ok ? 1 : 0;
     }
@@ -1061,13 +1063,30 @@ extern "C" int rdb_linear_projection_chunks(const rdb_linear_desc *d, int64_t *c
 
 static char *at_bytes(const void *p, int64_t bytes) { return static_cast<char *>(const_cast<void *>(p)) + bytes; }
 
+// Scratch that the projecting launches have a use for: that of the chunk that takes most.  It is not monotone in the tokens: the last chunk, with
+// fewer of them, has fewer tiles and so may have more ranges.
+static int64_t project_scratch(const rdb_linear_desc *d)
+{
+    if (f32_projected(d)) return check_desc("rdb_linear_workspace_bytes", d) ? 0 : linear_project_f32_scratch(d);
+    const ChunkPlan pl = chunk_plan(d);
+    if (pl.nchunks == 0) return 0;
+    const rdb_linear_desc first = chunk_desc(d, pl, 0), last = chunk_desc(d, pl, pl.nchunks - 1);
+    return std::max(linear_projection_scratch(&first), linear_projection_scratch(&last));
+}
+
 extern "C" int rdb_linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, void *stream)
+{
+    return rdb_linear_project_ws(state, x, ldx, coef, d, nullptr, 0, stream);
+}
+
+extern "C" int rdb_linear_project_ws(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, void *workspace,
+                                     int64_t workspace_bytes, void *stream)
 {
     if (f32_projected(d)) {
         if (int rc = check_projected_f32("rdb_linear_project", d)) return rc;
         if (!state || !x) return set_error(RDB_E_NULL, "rdb_linear_project: state or x is NULL");
         if (ldx < d->in_f) return set_error(RDB_E_SHAPE, "rdb_linear_project: leading dimension smaller than the row");
-        int rc = linear_project_f32(state, nullptr, 0, x, ldx, nullptr, nullptr, d, num_compute_units(), (hipStream_t)stream);
+        int rc = linear_project_f32(state, nullptr, 0, x, ldx, nullptr, nullptr, d, num_compute_units(), workspace, workspace_bytes, (hipStream_t)stream);
         if (rc == RDB_E_UNSUPPORTED) return set_error(RDB_E_UNSUPPORTED, "rdb_linear_project: state must be 16-byte aligned and tokens * ldx below 2^29");
         return rc;
     }
@@ -1081,7 +1100,8 @@ extern "C" int rdb_linear_project(void *state, const void *x, int64_t ldx, const
         return set_error(RDB_E_UNSUPPORTED, "rdb_linear_project: x and state must be 16-byte aligned, ldx a multiple of 8 and below twice in_f");
     for (int c = 0; c < pl.nchunks; ++c) {
         const rdb_linear_desc dd = chunk_desc(d, pl, c);
-        rc = linear_project(at_bytes(state, c * pl.state_stride), at_bytes(x, c * pl.chunk_tokens * ldx * 2), ldx, coef, &dd, (hipStream_t)stream);
+        rc = linear_project(at_bytes(state, c * pl.state_stride), at_bytes(x, c * pl.chunk_tokens * ldx * 2), ldx, coef, &dd, (hipStream_t)stream, workspace,
+                            workspace_bytes);
         if (rc == RDB_E_UNSUPPORTED) return set_error(RDB_E_UNSUPPORTED, "rdb_linear_project: internal: chunk %d of %d refused", c, pl.nchunks);
         if (rc) return rc;
     }
@@ -1121,11 +1141,17 @@ extern "C" int rdb_linear_fwd_projected(void *y, int64_t ldy, const void *z, con
 extern "C" int rdb_linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, const void *bias,
                                       const rdb_linear_desc *d, void *stream)
 {
+    return rdb_linear_project_fwd_ws(y, ldy, state, x, ldx, coef, bias, d, nullptr, 0, stream);
+}
+
+extern "C" int rdb_linear_project_fwd_ws(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, const void *bias,
+                                         const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
+{
     if (f32_projected(d)) {
         if (int rc = check_projected_f32("rdb_linear_project_fwd", d)) return rc;
         if (!y || !state || !x || !coef) return set_error(RDB_E_NULL, "rdb_linear_project_fwd: y, state, x or coef is NULL");
         if (ldx < d->in_f || ldy < d->out_f) return set_error(RDB_E_SHAPE, "rdb_linear_project_fwd: leading dimension smaller than the row");
-        int rc = linear_project_f32(state, y, ldy, x, ldx, coef, bias, d, num_compute_units(), (hipStream_t)stream);
+        int rc = linear_project_f32(state, y, ldy, x, ldx, coef, bias, d, num_compute_units(), workspace, workspace_bytes, (hipStream_t)stream);
         if (rc == RDB_E_UNSUPPORTED)
             return set_error(RDB_E_UNSUPPORTED, "rdb_linear_project_fwd: state must be 16-byte aligned and tokens * ldx, tokens * ldy below 2^29");
         return rc;
@@ -1142,7 +1168,8 @@ extern "C" int rdb_linear_project_fwd(void *y, int64_t ldy, void *state, const v
     for (int c = 0; c < pl.nchunks; ++c) {
         const rdb_linear_desc dd = chunk_desc(d, pl, c);
         rc = linear_project_fwd(at_bytes(y, c * pl.chunk_tokens * ldy * 2), ldy, at_bytes(state, c * pl.state_stride),
-                                at_bytes(x, c * pl.chunk_tokens * ldx * 2), ldx, coef, true, bias, &dd, num_compute_units(), (hipStream_t)stream);
+                                at_bytes(x, c * pl.chunk_tokens * ldx * 2), ldx, coef, true, bias, &dd, num_compute_units(), (hipStream_t)stream,
+                                SYNC_SPIN_LIMIT, workspace, workspace_bytes);
         if (rc == RDB_E_UNSUPPORTED) return set_error(RDB_E_UNSUPPORTED, "rdb_linear_project_fwd: internal: chunk %d of %d refused", c, pl.nchunks);
         if (rc) return rc;
     }
@@ -1154,22 +1181,29 @@ static int64_t project_fwd_rbias_table(const rdb_linear_desc *d)
     if (d->act_dtype != RDB_BF16 || d->coef_dtype != RDB_BF16 || d->sO != d->in_f || d->sI != 1 || chunk_plan(d).nchunks != 1) return 0;
     return rbias_big_table_bytes(d, d->out_f, num_compute_units());
 }
+// ... and behind R, from the next multiple of 256 on, the projection's scratch
+static int64_t project_fwd_rbias_bytes(const rdb_linear_desc *d)
+{
+    const int64_t table = project_fwd_rbias_table(d), more = table > 0 ? linear_projection_scratch(d) : 0;
+    return more > 0 ? (table + 255) / 256 * 256 + more : table;
+}
 
 extern "C" int rdb_linear_project_fwd_rbias(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, const void *scale_bias,
                                             const void *bias, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
 {
     const char *who = "rdb_linear_project_fwd_rbias";
     if (int rc = check_desc(who, d)) return rc;
-    const int64_t need = project_fwd_rbias_table(d);
+    const int64_t need = project_fwd_rbias_bytes(d);
     if (need <= 0) return set_error(RDB_E_UNSUPPORTED, "%s: a layer that has no such form (rdb_linear_workspace_bytes says 0)", who);
     if (!y || !x || !state || !coef || !scale_bias) return set_error(RDB_E_NULL, "%s: y, x, state, coef or scale_bias is NULL", who);
     if (ldy < d->out_f || ldx < d->in_f) return set_error(RDB_E_SHAPE, "%s: leading dimension smaller than the row", who);
     if (!workspace || workspace_bytes < need) return set_error(RDB_E_WORKSPACE, "%s: needs a workspace of %lld bytes", who, (long long)need);
     hipStream_t s = (hipStream_t)stream;
     int rc = RDB_E_UNSUPPORTED;
+    const int64_t table = (project_fwd_rbias_table(d) + 255) / 256 * 256;
     if (ldx % 8 == 0 && ldy % 8 == 0 && aligned16(x) && aligned16(y) && aligned16(state) && aligned16(coef) && aligned16(workspace) && !((uintptr_t)bias & 7) &&
         d->tokens * ldx < (1ll << 29) && d->tokens * ldy < (1ll << 29))
-        rc = linear_project_before(state, x, ldx, coef, y, ldy, d, num_compute_units(), s);
+        rc = linear_project_before(state, x, ldx, coef, y, ldy, d, num_compute_units(), s, at_bytes(workspace, table), workspace_bytes - table);
     if (!rc) rc = linear_fwd_rbias_big(y, ldy, x, ldx, state, coef, scale_bias, bias, d, workspace, num_compute_units(), s);
     if (rc == RDB_E_UNSUPPORTED)
         return set_error(rc, "%s: 16-byte aligned pointers (bias: 8-byte), leading dimensions multiples of 8, fewer than 2^29 elements per matrix", who);
@@ -1293,7 +1327,7 @@ extern "C" int rdb_linear_bwd_projected_to(void *dx, int64_t lddx, void *dcoef, 
 namespace rdb {   // rdb_f32.hip
 int64_t linear_kept_f32_bytes(const rdb_linear_desc *d);
 int linear_fwd_kept_f32(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias, const rdb_pseudo_bias *values,
-                        const rdb_linear_desc *d, int num_cus, hipStream_t s);
+                        const rdb_linear_desc *d, int num_cus, void *scratch, int64_t scratch_bytes, hipStream_t s);
 int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x, int64_t ldx,
                         const void *kept, const void *coef, const void *scale_bias, const rdb_linear_desc *d, int num_cus, void *workspace,
                         int64_t workspace_bytes, hipStream_t s);
@@ -1301,12 +1335,12 @@ int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, fl
 
 static bool kept_layer(const rdb_linear_desc *d)
 {
-    return !check_desc("rdb_linear_kept_bytes", d) && !rdb_linear_projection_preferred(d) && linear_kept_f32_z_bytes(d) > 0;
+    return !check_desc("rdb_linear_kept_bytes", d) && !rdb_linear_projection_preferred(d) && linear_kept_f32_bytes(d) > 0;
 }
 extern "C" int64_t rdb_linear_kept_bytes(const rdb_linear_desc *d) { return kept_layer(d) ? linear_kept_f32_bytes(d) : 0; }
 
 static int fwd_kept(const char *who, void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
-                    const rdb_pseudo_bias *values, const rdb_linear_desc *d, void *stream)
+                    const rdb_pseudo_bias *values, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
 {
     if (int rc = check_desc(who, d)) return rc;
     if (!kept_layer(d)) return set_error(RDB_E_UNSUPPORTED, "%s: a layer of which nothing is kept (rdb_linear_kept_bytes)", who);
@@ -1318,21 +1352,31 @@ static int fwd_kept(const char *who, void *y, int64_t ldy, void *kept, const voi
         if (d->act_dtype != RDB_F32 || values->k >= (1ll << 31) || d->out_f >= (1ll << 31))
             return set_error(RDB_E_UNSUPPORTED, "%s: fp32 layers, fewer than 2^31 coefficients and outputs", who);
     }
-    const int rc = linear_fwd_kept_f32(y, ldy, kept, x, ldx, coef, scale_bias, bias, values, d, num_compute_units(), (hipStream_t)stream);
+    const int rc = linear_fwd_kept_f32(y, ldy, kept, x, ldx, coef, scale_bias, bias, values, d, num_compute_units(), workspace, workspace_bytes,
+                                       (hipStream_t)stream);
     return rc == RDB_E_UNSUPPORTED ? set_error(rc, "%s: kept must be 16-byte aligned and tokens * ldx, tokens * ldy below 2^29", who) : rc;
 }
 
 extern "C" int rdb_linear_fwd_kept(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
                                    const rdb_linear_desc *d, void *stream)
 {
-    return fwd_kept("rdb_linear_fwd_kept", y, ldy, kept, x, ldx, coef, scale_bias, bias, nullptr, d, stream);
+    return fwd_kept("rdb_linear_fwd_kept", y, ldy, kept, x, ldx, coef, scale_bias, bias, nullptr, d, nullptr, 0, stream);
 }
 
 extern "C" int rdb_linear_fwd_kept_pseudo_bias(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias,
                                                const rdb_pseudo_bias *bias, const rdb_linear_desc *d, void *stream)
 {
     if (!bias) return set_error(RDB_E_NULL, "rdb_linear_fwd_kept_pseudo_bias: bias is NULL");
-    return fwd_kept("rdb_linear_fwd_kept_pseudo_bias", y, ldy, kept, x, ldx, coef, scale_bias, nullptr, bias, d, stream);
+    return fwd_kept("rdb_linear_fwd_kept_pseudo_bias", y, ldy, kept, x, ldx, coef, scale_bias, nullptr, bias, d, nullptr, 0, stream);
+}
+
+extern "C" int rdb_linear_fwd_kept_ws(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias,
+                                      const void *bias, const rdb_pseudo_bias *pseudo_bias, const rdb_linear_desc *d, void *workspace,
+                                      int64_t workspace_bytes, void *stream)
+{
+    const char *who = "rdb_linear_fwd_kept_ws";
+    if (bias && pseudo_bias) return set_error(RDB_E_SHAPE, "%s: one bias", who);
+    return fwd_kept(who, y, ldy, kept, x, ldx, coef, scale_bias, bias, pseudo_bias, d, workspace, workspace_bytes, stream);
 }
 
 extern "C" int rdb_linear_bwd_kept(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x,

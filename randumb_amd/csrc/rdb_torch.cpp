@@ -383,15 +383,19 @@ class OneCallLinear : public Function<OneCallLinear> {
         const Tensor c = coefs.contiguous(), sb = scale_bias ? scale_bias->to(c.scalar_type()) : Tensor();
         const Tensor xn = near_act(x);
         Tensor y = at::empty({x.size(0), l.out_f}, x.options()), kept = bytes(keep, x);
+        const int64_t room = rdb_linear_workspace_bytes(RDB_OP_LINEAR_FWD_KEPT, &d);
+        const Tensor ws = bytes(room, x);
+        auto call = [&](const Tensor &values, const rdb_pseudo_bias *pseudo) {
+            check(rdb_linear_fwd_kept_ws(y.data_ptr(), l.out_f, kept.data_ptr(), xn.data_ptr(), xn.stride(0), c.data_ptr(), ptr(sb), ptr(values), pseudo, &d, ptr(ws),
+                                         room, stream_of(x)),
+                  "rdb_linear_fwd_kept");
+        };
         if (b.beside(l.out_f, x.scalar_type())) {
             const Tensor bc = b.coef->contiguous(), bs = b.scale && b.scale->defined() ? b.scale->contiguous() : Tensor(), bv = at::empty({l.out_f}, x.options());
             const rdb_pseudo_bias pb = b.ref(bc, bs, bv);
-            check(rdb_linear_fwd_kept_pseudo_bias(y.data_ptr(), l.out_f, kept.data_ptr(), xn.data_ptr(), xn.stride(0), c.data_ptr(), ptr(sb), &pb, &d, stream_of(x)),
-                  "rdb_linear_fwd_kept");
+            call(Tensor(), &pb);
         } else {
-            const Tensor bv = b.values(l.out_f, x.scalar_type());
-            check(rdb_linear_fwd_kept(y.data_ptr(), l.out_f, kept.data_ptr(), xn.data_ptr(), xn.stride(0), c.data_ptr(), ptr(sb), ptr(bv), &d, stream_of(x)),
-                  "rdb_linear_fwd_kept");
+            call(b.values(l.out_f, x.scalar_type()), nullptr);
         }
         ctx->save_for_backward({scale_bias ? x0 : Tensor(), coefs, scale_bias.value_or(Tensor()), kept});
         return y;
@@ -482,7 +486,10 @@ class ProjectedLinear : public Function<ProjectedLinear> {
                                                one_product, s),
                   "rdb_linear_project_fwd_rbias");
         } else {
-            check(rdb_linear_project_fwd(y.data_ptr(), l.out_f, ptr(state), x.data_ptr(), x.stride(0), c.data_ptr(), ptr(b), &d, s), "rdb_linear_project_fwd");
+            const int64_t room = rdb_linear_workspace_bytes(RDB_OP_LINEAR_PROJECT, &d);
+            const Tensor ws = bytes(room, x);
+            check(rdb_linear_project_fwd_ws(y.data_ptr(), l.out_f, ptr(state), x.data_ptr(), x.stride(0), c.data_ptr(), ptr(b), &d, ptr(ws), room, s),
+                  "rdb_linear_project_fwd");
         }
         if (scale_bias && !one_product) {
             const Tensor sb = native(*scale_bias).to(at::kBFloat16);

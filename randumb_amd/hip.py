@@ -523,7 +523,7 @@ def _proj_desc(tokens, in_f, out_f, k, seed, coef_dtype=torch.bfloat16, act_dtyp
 
 class _ProjPlan:
     """What the projected calls need to know about a layer and batch, asked of the library once per (sizes, seed)."""
-    __slots__ = ("desc", "ref", "state_bytes", "state_cols", "ws_bytes", "ws_bytes_to", "chunks")
+    __slots__ = ("desc", "ref", "state_bytes", "state_cols", "project_bytes", "ws_bytes", "ws_bytes_to", "chunks")
 
     def __init__(self, tokens, in_f, out_f, k, seed, dtype):
         L = _lib.load()
@@ -531,6 +531,7 @@ class _ProjPlan:
         self.ref = ctypes.byref(self.desc)
         self.state_bytes = int(L.rdb_linear_projection_bytes(self.ref))
         self.state_cols = -(-self.state_bytes // tokens) if self.state_bytes > 0 else 0
+        self.project_bytes = int(L.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_PROJECT, self.ref))
         self.ws_bytes = int(L.rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_PROJECTED, self.ref))
         self.ws_bytes_to = int(L.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_BWD_PROJECTED_TO, self.ref))
         self.chunks = int(L.rdb_linear_projection_chunks(self.ref, None)) if self.state_bytes > 0 else 0
@@ -617,7 +618,9 @@ def linear_project(x: torch.Tensor, k: int, out_f: int, seed: int, coef: Optiona
         if tuple(c.shape) != (out_f, k):
             raise ValueError(f"coef must be ({out_f}, {k}), got {tuple(c.shape)}")
     with _on(x.device):
-        rc = L.rdb_linear_project(_p(state), _p(x), x.stride(0), _p(c), ctypes.byref(d), _stream(x.device))
+        ws_bytes = L.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_PROJECT, ctypes.byref(d))
+        ws = _workspace(ws_bytes, x.device)
+        rc = L.rdb_linear_project_ws(_p(state), _p(x), x.stride(0), _p(c), ctypes.byref(d), _p(ws), ws_bytes, _stream(x.device))
     _lib.check(rc, "rdb_linear_project")
     return state
 
@@ -643,8 +646,9 @@ def linear_project_fwd(x: torch.Tensor, coef: torch.Tensor, seed: int, bias: Opt
     y = torch.empty((tokens, out_f), dtype=x.dtype, device=dev)
     with _on(dev):
         st = _stream(dev)
-        rc = L.rdb_linear_project_fwd(y.data_ptr(), out_f, state.data_ptr(), x.data_ptr(), x.stride(0), c.data_ptr(),
-                                      None if b is None else b.data_ptr(), pl.ref, st)
+        ws = _workspace(pl.project_bytes, dev)
+        rc = L.rdb_linear_project_fwd_ws(y.data_ptr(), out_f, state.data_ptr(), x.data_ptr(), x.stride(0), c.data_ptr(),
+                                         None if b is None else b.data_ptr(), pl.ref, _p(ws), pl.project_bytes, st)
         if rc:
             _lib.check(rc, "rdb_linear_project_fwd")
         _watch(dev).tick(st)

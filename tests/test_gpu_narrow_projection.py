@@ -1,5 +1,5 @@
-"""Projection of layers whose y is too narrow for the sums of the contraction's ranges: they lie behind the state, where nothing is written
-over their tags, so replays of a graph on other inputs have to find them cleared."""
+"""Projection of layers whose y is too narrow for the sums of the contraction's ranges: they lie in scratch of the call's own, where nothing need be
+written over their tags, so replays of a graph on other inputs have to find them cleared."""
 import pytest
 import torch
 
@@ -73,22 +73,26 @@ def test_narrow_layers_in_fp32_sums(T, in_f, out_f, k, dtype, split):
     N = hip.sq5_fill_2d(in_f, k, 5).double()
     z = x.double() @ N
     want = z @ c.double().t()
-    calls = [("kept", lib.rdb_linear_kept_bytes(ref), 0)] + ([("state", lib.rdb_linear_projection_bytes(ref), 256)] if dtype is torch.float32 else [])
-    assert max(n for _, n, _ in calls) > 256 + (T * k * 4 + 255) // 256 * 256   # room for ranges
-    for what, n, at in calls:
+    calls = [("kept", lib.rdb_linear_kept_bytes(ref), 0, _lib.RDB_OP_LINEAR_FWD_KEPT)]
+    if dtype is torch.float32:
+        calls.append(("state", lib.rdb_linear_projection_bytes(ref), 256, _lib.RDB_OP_LINEAR_PROJECT))
+    rooms = [lib.rdb_linear_workspace_bytes(op, ref) for _, n, _, op in calls if n]
+    assert min(rooms) >= 3 * T * k * 4   # room for ranges
+    for what, n, at, op in calls:
         if n == 0:
             continue
-        kept = torch.full((n + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+        room = lib.rdb_linear_workspace_bytes(op, ref)
+        kept, ws = (torch.full((m + 64,), 0x5A, dtype=torch.uint8, device="cuda") for m in (n, room))
         y = torch.full((T + 1, out_f), 7.0, dtype=dtype, device="cuda")
         before = lib.rdb_set_f32_split(split)   # asked for after the buffer's size
         try:
             if what == "kept":
-                rc = lib.rdb_linear_fwd_kept(y.data_ptr(), out_f, kept.data_ptr(), x.data_ptr(), in_f, c.data_ptr(), None, None, ref, stream)
+                rc = lib.rdb_linear_fwd_kept_ws(y.data_ptr(), out_f, kept.data_ptr(), x.data_ptr(), in_f, c.data_ptr(), None, None, None, ref, ws.data_ptr(), room, stream)
             else:
-                rc = lib.rdb_linear_project_fwd(y.data_ptr(), out_f, kept.data_ptr(), x.data_ptr(), in_f, c.data_ptr(), None, ref, stream)
+                rc = lib.rdb_linear_project_fwd_ws(y.data_ptr(), out_f, kept.data_ptr(), x.data_ptr(), in_f, c.data_ptr(), None, ref, ws.data_ptr(), room, stream)
         finally:
             lib.rdb_set_f32_split(before)
-        assert rc == 0 and bool((kept[n:] == 0x5A).all()) and bool((y[T] == 7.0).all())
+        assert rc == 0 and bool((kept[n:] == 0x5A).all()) and bool((ws[room:] == 0x5A).all()) and bool((y[T] == 7.0).all())
         got = kept[at:at + T * k * 4].view(torch.float32).view(T, k).double()
         assert float((got - z).norm() / z.norm()) < 2e-6   # fp32 sums of products of fp32 accuracy
         # y rounded once: to bf16 2^-9 at most

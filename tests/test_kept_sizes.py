@@ -1,0 +1,45 @@
+"""What a layer keeps from its forward to its backward pass: z and, in bf16, the transposed coefficients; scratch of the forward pass is asked for apart."""
+import ctypes
+import random
+
+import pytest
+
+from randumb_amd import _lib
+
+
+def _desc(tokens, in_f, out_f, k, dtype):
+    d = _lib.LinearDesc()
+    d.tokens, d.in_f, d.out_f, d.k, d.coef_rows, d.sO, d.sI, d.seed = tokens, in_f, out_f, k, out_f, in_f, 1, 5
+    d.act_dtype = d.coef_dtype = dtype
+    d.algo = _lib.RDB_ALGO_AUTO
+    return d
+
+
+def _up(n, to=256):
+    return -(-n // to) * to
+
+
+# narrow layers, whose projection runs in ranges that y has no room for, among layers of any shape
+CASES = [(2048, 3072, 768, 256), (256, 8192, 1024, 512), (257, 8192, 1024, 32), (700, 4000, 256, 120), (492, 3184, 273, 118), (433, 3320, 96, 144)]
+
+
+@pytest.mark.parametrize("dtype", [_lib.RDB_BF16, _lib.RDB_F32])
+def test_nothing_but_what_the_backward_pass_reads(dtype):
+    lib, rng = _lib.load(), random.Random(3)
+    cases = CASES + [tuple(int(2 ** rng.uniform(*r)) for r in ((5, 13), (3, 13), (0, 12), (3, 9))) for _ in range(3000)]
+    scratch = 0
+    for T, in_f, out_f, k in cases:
+        ref = ctypes.byref(_desc(T, in_f, out_f, k, dtype))
+        state, kept = lib.rdb_linear_projection_bytes(ref), lib.rdb_linear_kept_bytes(ref)
+        assert kept in (0, _up(4 * T * k)), (T, in_f, out_f, k)
+        if dtype == _lib.RDB_F32:
+            assert state == 256 + _up(4 * T * k), (T, in_f, out_f, k)
+        elif state:
+            kpad = _up(k, 64)
+            z, z_t, c_t, tags = (_up(n) for n in (_up(T, 32) * kpad * 2, _up(T, 64) * kpad * 2, _up(out_f, 64) * kpad * 2, -(-T // 256) * (kpad // 32 + 1) * 8))
+            assert state == 256 + z + z_t + c_t + tags, (T, in_f, out_f, k)
+        for op, has in ((_lib.RDB_OP_LINEAR_PROJECT, state), (_lib.RDB_OP_LINEAR_FWD_KEPT, kept)):
+            n = lib.rdb_linear_workspace_bytes(op, ref)
+            assert 0 <= n <= 33 << 20 and (has or n == 0), (T, in_f, out_f, k, op)
+            scratch += n > 0
+    assert scratch > 20

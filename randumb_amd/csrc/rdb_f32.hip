@@ -137,20 +137,37 @@ static int z_room(const rdb_linear_desc *d, int num_cus)
 static int t_room(const rdb_linear_desc *d, int num_cus) { return fg_room(d->tokens, d->k, d->out_f, num_cus, 128, 32).ranges; }
 static int dc_room(const rdb_linear_desc *d, int num_cus) { return fg_room(d->out_f, d->k, d->tokens, num_cus, 256, 64).ranges; }
 
+// z's ranges that a workspace is asked for: those that pay, whichever products are on (rdb_set_f32_split).  All that z_room allows is up to twice that
+// (2048 x 768, k = 256: 27.3 MB instead of 14.7).
+static double z_host_us(const rdb_linear_desc *d);
+static int z_ranges(const rdb_linear_desc *d, int num_cus)
+{
+    const int room = z_room(d, num_cus);
+    if (room <= 1 || d->tokens < 32) return room;
+    auto ranges = [&](bool split) { return fg_plan(d->tokens, d->k, d->in_f, num_cus, room, FgGroups<FG_KCONT, FG_NOISE_M>::four, z_host_us(d), split).ranges; };
+    return std::max(ranges(true), ranges(false));
+}
+static int64_t with_parts(const rdb_linear_desc *d, int ranges) { return up256(d->tokens * d->k * 4) * (ranges > 1 ? 1 + ranges : 1); }
+
 // scratch: z or t [tokens x k] and its partial matrices; for the coefficient gradient also one [out_f x k] matrix per token range
 int64_t linear_f32_workspace(int op, const rdb_linear_desc *d, int num_cus)
 {
     rdb_linear_desc dd = *d;
     if (op == RDB_OP_LINEAR_BWD_DCOEF) dd.coef_dtype = dd.act_dtype;   // reads no coefficients
     if (!fg_ok(&dd)) return 0;
-    const int64_t zt = up256(d->tokens * d->k * 4);
-    auto with_parts = [&](int r) { return zt * (r > 1 ? 1 + r : 1); };
-    if (op == RDB_OP_LINEAR_FWD) return with_parts(z_room(d, num_cus));
-    if (op == RDB_OP_LINEAR_BWD_DX) return with_parts(t_room(d, num_cus));
+    if (op == RDB_OP_LINEAR_FWD) return with_parts(d, z_ranges(d, num_cus));
+    if (op == RDB_OP_LINEAR_BWD_DX) return with_parts(d, t_room(d, num_cus));
     if (op != RDB_OP_LINEAR_BWD_DCOEF) return 0;
     const int r = dc_room(d, num_cus);
     // ... and, for the gradient of the random bias's scale, one value per 64 x 128 tile of [tokens x out_f]
-    return with_parts(z_room(d, num_cus)) + (r > 1 ? (int64_t)r * up256(d->out_f * d->k * 4) : 0) + up256(cdiv(d->tokens, 64) * cdiv(d->out_f, FG_BN) * 4);
+    return with_parts(d, z_ranges(d, num_cus)) + (r > 1 ? (int64_t)r * up256(d->out_f * d->k * 4) : 0) + up256(cdiv(d->tokens, 64) * cdiv(d->out_f, FG_BN) * 4);
+}
+
+// The forward pass runs with room for ranges of 128 values and more, in as many as there is room for: shorter ones may pay, and are not needed.
+int64_t linear_f32_fwd_workspace_least(const rdb_linear_desc *d, int num_cus)
+{
+    if (!fg_ok(d)) return 0;
+    return with_parts(d, std::min(z_ranges(d, num_cus), fg_room(d->tokens, d->k, d->in_f, num_cus, 128, 32).ranges));
 }
 
 static bool fg_ws_ok(int op, const rdb_linear_desc *d, int num_cus, const void *ws, int64_t bytes)
@@ -213,7 +230,7 @@ static int fg_launch_pair_ranges(FgProduct t, int t_room, float *t_part, int64_t
     return fg_launch_sums(sum[0], sum[1], s);
 }
 
-// What z's launch of sums counts for on the host: nothing where the step's products, z, y, t, dC and dx at 1.16 PFLOP/s, take 40 us and more (with as much
+// What z's launch of sums counts for on the host (z_ranges): nothing where the step's products, z, y, t, dC and dx at 1.16 PFLOP/s, take 40 us and more (with as much
 // again for what they wait, the kernels then outlast the host's 60 to 70: 2859 tokens x 584 -> 7920, k = 208, step 219 us, 222 with z in one range).
 static double z_host_us(const rdb_linear_desc *d)
 {
@@ -264,10 +281,11 @@ static int fg_project_kept(float *z, const void *x, int64_t ldx, void *y, int64_
 int linear_fwd_f32(void *y, int64_t ldy, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
                    const rdb_linear_desc *d, int num_cus, void *workspace, int64_t workspace_bytes, hipStream_t s)
 {
-    if (!fg_ok(d) || !fg_wanted(d) || !fg_ws_ok(RDB_OP_LINEAR_FWD, d, num_cus, workspace, workspace_bytes)) return RDB_E_UNSUPPORTED;
+    if (!fg_ok(d) || !fg_wanted(d) || !workspace || !fg_aligned16(workspace) || workspace_bytes < linear_f32_fwd_workspace_least(d, num_cus)) return RDB_E_UNSUPPORTED;
     if (d->tokens * ldx >= (1ll << 29) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     float *z = (float *)workspace;
-    if (int rc = fg_project(z, (const float *)x, ldx, d, num_cus, s)) return rc;
+    const int64_t parts = workspace_bytes / up256(d->tokens * d->k * 4) - 1;
+    if (int rc = fg_project(z, (const float *)x, ldx, d, num_cus, s, nullptr, (int)std::min<int64_t>(parts, z_ranges(d, num_cus)))) return rc;
     FgProduct q = {z, d->k, d->tokens * d->k, (const float *)coef, d->k, d->out_f * d->k, (float *)y, ldy, (const float *)bias,
                    d->tokens, d->out_f, d->k, 0, 0, 0, 0, d->seed};
     const int b16 = d->act_dtype == RDB_BF16;
@@ -365,8 +383,8 @@ int linear_dcoef_f32(float *dcoef, float *d_scale_bias, const void *dy, int64_t 
     if (!fg_ok(&dd) || !fg_wanted(&dd) || !fg_ws_ok(RDB_OP_LINEAR_BWD_DCOEF, &dd, num_cus, workspace, workspace_bytes)) return RDB_E_UNSUPPORTED;
     if (d->tokens * ldx >= (1ll << 29) || d->tokens * lddy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     float *z = (float *)workspace;
-    if (int rc = fg_project(z, (const float *)x, ldx, &dd, num_cus, s)) return rc;
-    const int zs = z_room(&dd, num_cus);
+    const int zs = z_ranges(&dd, num_cus);
+    if (int rc = fg_project(z, (const float *)x, ldx, &dd, num_cus, s, nullptr, zs)) return rc;
     float *part = reinterpret_cast<float *>(static_cast<char *>(workspace) + up256(d->tokens * d->k * 4) * (zs > 1 ? 1 + zs : 1));
     const int dcr = dc_room(&dd, num_cus);
     if (int rc = fg_launch_ranges<FG_MCONT, FG_MCONT>(fg_dc(dcoef, RDB_F32, dy, lddy, z, &dd), dcr, part, up256(d->out_f * d->k * 4) / 4, num_cus, s, "f32_gemm_kernel (dC = dy^T . z)")) return rc;

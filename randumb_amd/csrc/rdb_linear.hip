@@ -316,6 +316,7 @@ int num_compute_units();   // of the current device (256 when there is none)
 
 // rdb_f32.hip
 int64_t linear_f32_workspace(int op, const rdb_linear_desc *d, int num_cus);
+int64_t linear_f32_fwd_workspace_least(const rdb_linear_desc *d, int num_cus);
 int linear_fwd_f32(void *y, int64_t ldy, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
                    const rdb_linear_desc *d, int num_cus, void *workspace, int64_t workspace_bytes, hipStream_t s);
 bool f32_products_first(const rdb_linear_desc *d, bool dx);   // ahead of the few-token kernels
@@ -917,13 +918,22 @@ static int static_scratch_ptr(void **out)
 
 extern "C" int64_t rdb_linear_fwd_static_max_bytes(void) { return RDB_STATIC_SCRATCH_BYTES; }
 
+// How much of the forward pass's workspace its kernels can do without
+static int64_t fwd_workspace_spare(const rdb_linear_desc *d)
+{
+    const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_FWD, d);
+    if (need == linear_projection_bytes(d) + linear_projection_scratch(d)) return linear_projection_scratch(d);
+    const int num_cus = num_compute_units();
+    return need == linear_f32_workspace(RDB_OP_LINEAR_FWD, d, num_cus) ? need - linear_f32_fwd_workspace_least(d, num_cus) : 0;
+}
+
 extern "C" int rdb_linear_fwd_static(void *y, int64_t ldy, const void *x, int64_t ldx, const void *coef, const void *scale_bias,
                                      const void *bias, const rdb_linear_desc *d, void *stream)
 {
     int rc = check_desc("rdb_linear_fwd_static", d);
     if (rc) return rc;
     int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_FWD, d);
-    if (need > RDB_STATIC_SCRATCH_BYTES && need == linear_projection_bytes(d) + linear_projection_scratch(d)) need = linear_projection_bytes(d);   // goes without
+    if (need > RDB_STATIC_SCRATCH_BYTES) need -= fwd_workspace_spare(d);   // ranges of the projection run one after the other, or fewer of them
     if (need > RDB_STATIC_SCRATCH_BYTES)
         return set_error(RDB_E_WORKSPACE, "rdb_linear_fwd_static: this layer's kernels use %lld bytes of scratch, the library's static scratch holds "
                                           "%lld: call rdb_linear_fwd with a workspace of the caller's", (long long)need, (long long)RDB_STATIC_SCRATCH_BYTES);

@@ -82,3 +82,23 @@ def test_static_scratch_rejects_what_does_not_fit():
     d = _desc(65536, 768, 3072, 256, 0)     # 64 MiB of projection state
     rc = L.rdb_linear_fwd_static(ctypes.c_void_p(256), 3072, ctypes.c_void_p(256), 768, ctypes.c_void_p(256), None, None, ctypes.byref(d), None)
     assert rc == -6 and b"static scratch holds" in L.rdb_last_error_string()
+
+
+# fp32 sums near the line: more ranges of the projection would pay than the static array has room for beside z, and the layer goes without them
+@pytest.mark.parametrize("tokens,in_f,out_f,k,dtype", [(2048, 768, 264, 256, torch.float32), (1024, 1024, 136, 256, torch.float32), (512, 2048, 72, 256, torch.float32),
+                                                       (4097, 1001, 333, 100, torch.bfloat16)])
+def test_static_scratch_takes_layers_that_could_use_more(tokens, in_f, out_f, k, dtype):
+    from randumb_amd import hip
+
+    print(f"case static scratch near the line {tokens} x {in_f} -> {out_f}, k = {k}, {dtype}", flush=True)
+    L, vp = _lib.load(), ctypes.c_void_p
+    g = torch.Generator().manual_seed(tokens)
+    x, C = torch.randn(tokens, in_f, generator=g).to(dtype).cuda(), (torch.randn(out_f, k, generator=g) / k ** 0.5).to(dtype).cuda()
+    r, stream, size = ctypes.byref(_desc(tokens, in_f, out_f, k, 5, dtype)), vp(torch.cuda.current_stream().cuda_stream), L.rdb_linear_fwd_static_max_bytes()
+    y, y_ref = (torch.full((tokens, out_f), float("nan"), dtype=dtype, device="cuda") for _ in range(2))
+    _lib.check(L.rdb_linear_fwd_static(vp(y.data_ptr()), out_f, vp(x.data_ptr()), in_f, vp(C.data_ptr()), None, None, r, stream), "rdb_linear_fwd_static")
+    ws = torch.full((size + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+    _lib.check(L.rdb_linear_fwd(vp(y_ref.data_ptr()), out_f, vp(x.data_ptr()), in_f, vp(C.data_ptr()), None, None, r, vp(ws.data_ptr()), size, stream), "rdb_linear_fwd")
+    assert torch.equal(y, y_ref) and bool((ws[size:] == 0x5A).all())
+    want = x.double() @ hip.sq5_fill_2d(in_f, k, 5).double() @ C.double().t()
+    assert float((y.double() - want).norm() / want.norm()) < (2.0 ** -9 if dtype is torch.bfloat16 else 4e-6)   # fp32 sums; y rounded once to bf16

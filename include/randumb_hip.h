@@ -391,7 +391,7 @@ int64_t rdb_linear_kept_bytes(const rdb_linear_desc *desc);
 int rdb_linear_fwd_kept(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef,
                         const void *scale_bias, const void *bias, const rdb_linear_desc *desc, void *stream);
 /* The same for an fp32 layer with a pseudorandom bias, b[o] = sum_m noise(PRIME*o + m) coef[m] (+ scale[0] noise1d(o)): its values (out_f
- * floats, overwritten) are formed beside the projection, in the same launch.  RDB_E_UNSUPPORTED: another dtype, k or out_f of 2^31 or more. */
+ * floats, overwritten) are formed beside the projection, in the same launch where they are few and their sums short.  RDB_E_UNSUPPORTED: another dtype, k or out_f of 2^31 or more. */
 int rdb_linear_fwd_kept_pseudo_bias(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef,
                                     const void *scale_bias, const rdb_pseudo_bias *bias, const rdb_linear_desc *desc, void *stream);
 /* Both (bias or pseudo_bias, or neither) with scratch for the projection as in rdb_linear_project_ws:

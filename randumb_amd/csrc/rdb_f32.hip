@@ -451,16 +451,19 @@ static int fg_rbias(FgProduct q, const void *scale, const rdb_linear_desc *d, in
     return fg_launch<FG_KCONT, FG_NOISE_1D>(q, num_cus, s, name);
 }
 
-// values: NULL, or a pseudorandom bias whose values the launch of the projection forms on the side (an fp32 layer's; then `bias`)
+// values: NULL, or a pseudorandom bias whose values the launch of the projection forms on the side, or one of their own (an fp32 layer's; then `bias`)
 int linear_fwd_kept_f32(void *y, int64_t ldy, void *kept, const void *x, int64_t ldx, const void *coef, const void *scale_bias, const void *bias,
                         const rdb_pseudo_bias *values, const rdb_linear_desc *d, int num_cus, void *scratch, int64_t scratch_bytes, hipStream_t s)
 {
+    if (!linear_kept_f32_bytes(d) || !fg_aligned16(kept) || d->tokens * ldx >= (1ll << 29) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     FgValues v = {};
     if (values) {
-        v = {values->values, values->coef, values->scale, (int)d->out_f, (int)values->k, values->seed};
         bias = values->values;
+        if (values->k <= FG_VALUES_K && d->out_f <= FG_VALUES_N)
+            v = {values->values, values->coef, values->scale, (int)d->out_f, (int)values->k, values->seed, 0};
+        else if (int rc = rdb_materialize_fwd(values->values, values->coef, RDB_F32, 0, values->k, 0, 1, d->out_f, 0, 1, values->seed, values->scale, (void *)s))
+            return rc;
     }
-    if (!linear_kept_f32_bytes(d) || !fg_aligned16(kept) || d->tokens * ldx >= (1ll << 29) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     float *z = static_cast<float *>(kept);
     if (int rc = fg_project_kept(z, x, ldx, y, ldy, d, num_cus, scratch, scratch_bytes, s, v)) return rc;
     FgProduct q = {z, d->k, d->tokens * d->k, (const float *)coef, d->k, d->out_f * d->k, (float *)y, ldy, (const float *)bias, d->tokens, d->out_f, d->k,

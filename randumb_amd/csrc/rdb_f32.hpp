@@ -37,6 +37,7 @@ struct FgValues {
     const float *coef, *scale;   // scale: NULL, or one value
     int n, k;                    // n: 0: no such blocks
     uint32_t seed;
+    int slices;                  // of the launch's grid along z, behind the product's
 };
 __device__ __forceinline__ void fg_values(const FgValues &v, int thread, int threads)
 {
@@ -54,6 +55,21 @@ __device__ __forceinline__ void fg_values(const FgValues &v, int thread, int thr
         if (part == 0) v.out[e] = v.scale ? acc + v.scale[0] * noise1d((uint32_t)e, v.seed) : acc;
     }
 }
+
+// As many blocks as leave a thread 16 hashes, or one element's: the product's tiles may be a single one, and with one block for each of them 64 tokens x
+// 4096 -> 4096, k = 64, a bias of 64 coefficients took 57 us (now 19.3, without a bias 18.8), -> 32768 518 (now 15.9, without 15.2).  32 hashes: 17.9 -> 19.2 for
+// 128 x 2048 -> 2048, and 64 24.6; 8: the same.
+constexpr int FG_VALUE_HASHES = 16;
+inline int fg_value_slices(const FgValues &v, int64_t tiles, int threads)
+{
+    if (!v.n) return 0;
+    const int64_t each = std::max<int64_t>(1, FG_VALUE_HASHES / std::max<int64_t>(1, cdiv(v.k, 16)));   // elements of sixteen lanes
+    return (int)cdiv(cdiv(cdiv(v.n, each) * 16, threads), tiles);
+}
+// Beside the projection up to 64 hashes a lane in turn: more are longer than its blocks run, and a launch of its own, with more waves to a unit, ends sooner
+// (us, beside and apart: 128 x 2048 -> 2048 with 64 coefficients 17.9, 20.3; 1024 22.4, 23.9; 1536 26.8, 26.0; 4096 47.4, 37.1; 64 x 784 -> 32768 with 1024 33.4,
+// 34.3); n: of the tensors that a launch of their own adds up in the same order.
+constexpr int FG_VALUES_K = 1024, FG_VALUES_N = 1 << 15;
 
 struct FgParams {
     const float *a;   // A operand's matrix (FG_KCONT / FG_MCONT)
@@ -711,9 +727,11 @@ __global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kerne
     __shared__ __align__(16) float lds[FgBlock<BM, G, ASRC, BSRC, VEC, SPLIT, AES, BES>::LDS];
     __shared__ int not_finite;   // some thread's sum is an infinity or a NaN
     if constexpr (BSRC == FG_NOISE_M) {
-        if (p.values.n && blockIdx.z == gridDim.z - 1) {
+        const unsigned products = gridDim.z - (unsigned)p.values.slices;
+        if (blockIdx.z >= products) {
             constexpr int THREADS = FG_THREADS * G;
-            fg_values(p.values, (int)(blockIdx.y * gridDim.x + blockIdx.x) * THREADS + (int)threadIdx.x, (int)(gridDim.x * gridDim.y) * THREADS);
+            const int tiles = (int)(gridDim.x * gridDim.y), block = (int)(blockIdx.z - products) * tiles + (int)(blockIdx.y * gridDim.x + blockIdx.x);
+            fg_values(p.values, block * THREADS + (int)threadIdx.x, p.values.slices * tiles * THREADS);
             return;
         }
     }
@@ -986,12 +1004,13 @@ template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_
         q.groups = pl.groups;
     }
     if (!fg_fits(q)) return RDB_E_UNSUPPORTED;
+    if constexpr (BSRC == FG_NOISE_M) q.values.slices = fg_value_slices(q.values, cdiv(q.M, q.bm) * cdiv(q.N, FG_BN), FG_THREADS * (q.split ? q.groups : 1));
     const FgParams p = fg_params(q);
     const int splits = (int)cdiv(q.K, p.kchunk);
     const bool vec = fg_vec(q, ASRC, BSRC);
     const bool a16 = (ASRC == FG_KCONT || ASRC == FG_MCONT) && q.a_es == 2, b16 = (BSRC == FG_KCONT || BSRC == FG_MCONT) && q.b_es == 2;
     if (q.split && ((a16 && b16) ? !Groups::a16_b16 : a16 ? !Groups::a16_b32 : b16 && !Groups::a32_b16)) return RDB_E_UNSUPPORTED;
-    const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)(splits + (BSRC == FG_NOISE_M && q.values.n ? 1 : 0)));
+    const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)(splits + (BSRC == FG_NOISE_M ? q.values.slices : 0)));
     auto run = [&](auto epi_) {
         constexpr int EPI = decltype(epi_)::value;
         if (q.bm == 128 && q.groups == 2) FG_LAUNCH_GROUPS(128, 2, EPI);

@@ -33,8 +33,10 @@ def test_weight_and_bias(n, k, bn, bk, scaled):
     assert bool((w[n:] == 7.0).all()) and bool((b[bn:] == 7.0).all())
 
 
-# one tile and many, more elements than the launch has groups of lanes, ranges of the contraction beside them
-@pytest.mark.parametrize("T,in_f,out_f,k,bk", [(64, 784, 256, 64, 64), (33, 301, 1, 7, 8), (128, 256, 10, 64, 64), (32, 512, 4099, 96, 130)])
+# one tile and many, one slice of the grid and many, more elements than a slice has groups of lanes, ranges of the contraction beside them; the longest sums
+# and the most elements that are formed beside the projection, and one more of each
+@pytest.mark.parametrize("T,in_f,out_f,k,bk", [(64, 784, 256, 64, 64), (33, 301, 1, 64, 8), (128, 256, 10, 64, 64), (32, 512, 4099, 96, 130), (64, 4096, 4099, 64, 17),
+                                               (700, 264, 301, 40, 33), (64, 784, 1000, 64, 1024), (64, 784, 77, 64, 1025), (64, 784, 32768, 64, 9), (64, 784, 32769, 64, 9)])
 @pytest.mark.parametrize("scaled", [False, True])
 @pytest.mark.parametrize("split", [1, 0])
 def test_layer(T, in_f, out_f, k, bk, scaled, split):
@@ -46,8 +48,7 @@ def test_layer(T, in_f, out_f, k, bk, scaled, split):
     x, c, bc, s = (torch.randn(*m, generator=g).cuda() for m in ((T, in_f), (out_f, k), (bk,), (1,)))
     ref = ctypes.byref(hip._desc(T, in_f, out_f, c, in_f, 1, 5, torch.float32, 0))
     size = lib.rdb_linear_kept_bytes(ref)
-    if not size:
-        pytest.skip("a layer of which nothing is kept")
+    assert size > 0
     before = lib.rdb_set_f32_split(split)
     try:
         sc, values = s if scaled else None, torch.full((out_f + 4,), 7.0, device="cuda")
@@ -61,3 +62,24 @@ def test_layer(T, in_f, out_f, k, bk, scaled, split):
         assert torch.equal(y, want) and torch.equal(kept, want_kept)
     finally:
         lib.rdb_set_f32_split(before)
+
+
+def test_many_values_beside_few_tiles():
+    """A projection of a single tile of rows beside 32768 values: one block a tile formed them all in 500 us, where the layer without a bias takes 16."""
+    from randumb_amd import SillyLinear
+
+    print("case a long bias beside few tiles", flush=True)
+    x, us = torch.randn(64, 784, device="cuda").requires_grad_(), []
+    for bias in (True, False):
+        layer = SillyLinear(784, 32768, [64, 64], [1, 2], bias=bias, device="cuda", matrix_coef=True)
+        best = 1e9
+        for _ in range(20):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(10):
+                layer(x)
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end) * 100.0)
+        us.append(best)
+    assert us[0] < us[1] + 100.0, us

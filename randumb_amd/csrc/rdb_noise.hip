@@ -960,6 +960,10 @@ extern "C" int rdb_bias_bwd(float *dcoef, float *ds, const void *dy, int dtype, 
     float *part = static_cast<float *>(workspace);
     int chunks = bias_chunks(rows);
     const int64_t blocks = (dcoef ? cdiv(k, BIAS_M) : 0) + (ds ? 1 : 0);
+    // asked for whichever kernels run
+    if (n > 0 && (!workspace || ((uintptr_t)workspace & 3) || workspace_bytes < rdb_bias_bwd_workspace_bytes(rows, n)))
+        return set_error(RDB_E_WORKSPACE, "rdb_bias_bwd: workspace of %lld bytes needed, %lld given", (long long)rdb_bias_bwd_workspace_bytes(rows, n),
+                         (long long)workspace_bytes);
     if (bias_direct(rows, n, dtype == RDB_BF16 ? 2 : 4)) {
         const int wide = bias_wide(n);
         if (dtype == RDB_BF16) bias_grad_direct_kernel<bf16_t><<<(unsigned)blocks, 1024, 0, s>>>(dcoef, ds, static_cast<const bf16_t *>(dy), ldy, (int)rows, (int)n, wide, k, seed);
@@ -967,9 +971,6 @@ extern "C" int rdb_bias_bwd(float *dcoef, float *ds, const void *dy, int dtype, 
         return check_launch("bias_grad_direct_kernel");
     }
     if (n > 0) {
-        if (!workspace || ((uintptr_t)workspace & 3) || workspace_bytes < rdb_bias_bwd_workspace_bytes(rows, n))
-            return set_error(RDB_E_WORKSPACE, "rdb_bias_bwd: workspace of %lld bytes needed, %lld given", (long long)rdb_bias_bwd_workspace_bytes(rows, n),
-                             (long long)workspace_bytes);
         const int64_t per = cdiv(rows, chunks);
         const int es = dtype == RDB_BF16 ? 2 : 4, V = 16 / es;
         const bool vec = ((uintptr_t)dy & 15) == 0 && ldy % V == 0 && n % V == 0;

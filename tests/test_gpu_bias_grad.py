@@ -30,3 +30,15 @@ def test_against_float64(rows, n, k, dtype):
     alone = [t.clone() for t in (dc, ds)]
     assert call(alone[0].data_ptr(), 0) == 0 and call(0, alone[1].data_ptr()) == 0
     assert torch.equal(alone[0], dc) and torch.equal(alone[1], ds)
+
+
+@pytest.mark.parametrize("rows,n", [(128, 10), (65, 1024)])
+def test_a_workspace_is_asked_for_whichever_kernels_run(rows, n):
+    from randumb_amd import _lib
+
+    print(f"case bias gradient without its workspace {rows} x {n}", flush=True)
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    dy, dc, need = torch.randn(rows, n, device="cuda"), torch.empty(8, device="cuda"), lib.rdb_bias_bwd_workspace_bytes(rows, n)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    call = lambda w, size: lib.rdb_bias_bwd(dc.data_ptr(), 0, dy.data_ptr(), 0, n, rows, n, 8, 11, w, size, stream)
+    assert call(0, need) == -6 and call(ws.data_ptr(), need - 1) == -6 and call(ws.data_ptr(), need) == 0

@@ -890,13 +890,15 @@ template <int THREADS> __device__ __forceinline__ void bias_finish(float (&acc)[
 
 // The whole gradient in one launch, for a dy so small that every block may read it: blocks of 1024 threads, as many of them side by side
 // on a column's rows as its outputs leave room for, sixteen rows in flight each.  3.3 us and 1.3 for every sixteen rows of a thread, against
-// 8.2 (and a launch more on the host) for the two: 128 rows x 256 5.9, 128 x 10 4.6, 512 x 128 8.5; 250 x 262, six turns, 11.0.
+// 8.2 (and a launch more on the host) for the two: 128 rows x 256 5.9, 128 x 10 4.6, 512 x 128 8.5; 250 x 262, six turns, 11.0.  Only while a
+// compute unit has one block, which reads all of dy, whichever gradients are wanted (512 x 128: k = 1016 8.7, 1024 13.2, 4096 29.5, 16384 94, and the two
+// launches there 6.0, 6.0, 6.3 and 10 behind one another).
 constexpr int64_t BIAS_DIRECT_BYTES = 256 << 10, BIAS_DIRECT_TURNS = 4;
 constexpr int BIAS_AHEAD = 16;
 static int bias_wide(int64_t n) { return n < 1024 ? (int)cdiv(n, 64) * 64 : 1024; }   // threads along the outputs
-static bool bias_direct(int64_t rows, int64_t n, int es)
+static bool bias_direct(int64_t rows, int64_t n, int es, int64_t k)
 {
-    if (rows <= 0 || n <= 0 || rows * n * es > BIAS_DIRECT_BYTES) return false;
+    if (rows <= 0 || n <= 0 || rows * n * es > BIAS_DIRECT_BYTES || cdiv(k, BIAS_M) + 1 > num_compute_units()) return false;
     const int wide = bias_wide(n);
     return cdiv(rows, BIAS_AHEAD * (1024 / wide)) * cdiv(n, wide) <= BIAS_DIRECT_TURNS;
 }
@@ -964,7 +966,7 @@ extern "C" int rdb_bias_bwd(float *dcoef, float *ds, const void *dy, int dtype, 
     if (n > 0 && (!workspace || ((uintptr_t)workspace & 3) || workspace_bytes < rdb_bias_bwd_workspace_bytes(rows, n)))
         return set_error(RDB_E_WORKSPACE, "rdb_bias_bwd: workspace of %lld bytes needed, %lld given", (long long)rdb_bias_bwd_workspace_bytes(rows, n),
                          (long long)workspace_bytes);
-    if (bias_direct(rows, n, dtype == RDB_BF16 ? 2 : 4)) {
+    if (bias_direct(rows, n, dtype == RDB_BF16 ? 2 : 4, k)) {
         const int wide = bias_wide(n);
         if (dtype == RDB_BF16) bias_grad_direct_kernel<bf16_t><<<(unsigned)blocks, 1024, 0, s>>>(dcoef, ds, static_cast<const bf16_t *>(dy), ldy, (int)rows, (int)n, wide, k, seed);
         else bias_grad_direct_kernel<float><<<(unsigned)blocks, 1024, 0, s>>>(dcoef, ds, static_cast<const float *>(dy), ldy, (int)rows, (int)n, wide, k, seed);

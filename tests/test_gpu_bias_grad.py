@@ -5,8 +5,10 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# one output, one row, as many threads side by side as there are, none beside, outputs past one turn of the block, just past the line
-@pytest.mark.parametrize("rows,n,k", [(1, 1, 1), (128, 10, 64), (17, 64, 5), (511, 65, 33), (64, 1000, 16), (33, 1025, 7), (1, 4097, 3), (64, 1024, 8), (65, 1024, 8)])
+# one output, one row, as many threads side by side as there are, none beside, outputs past one turn of the block, just past the line;
+# as many coefficients as a block a compute unit takes, and one more
+@pytest.mark.parametrize("rows,n,k", [(1, 1, 1), (128, 10, 64), (17, 64, 5), (511, 65, 33), (64, 1000, 16), (33, 1025, 7), (1, 4097, 3), (64, 1024, 8), (65, 1024, 8),
+                                      (40, 70, 1020), (40, 70, 1021)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_against_float64(rows, n, k, dtype):
     from randumb_amd import _lib, hip
@@ -42,3 +44,25 @@ def test_a_workspace_is_asked_for_whichever_kernels_run(rows, n):
     ws = torch.empty(need, dtype=torch.uint8, device="cuda")
     call = lambda w, size: lib.rdb_bias_bwd(dc.data_ptr(), 0, dy.data_ptr(), 0, n, rows, n, 8, 11, w, size, stream)
     assert call(0, need) == -6 and call(ws.data_ptr(), need - 1) == -6 and call(ws.data_ptr(), need) == 0
+
+
+def test_many_coefficients():
+    """512 x 128, which one launch takes with few coefficients, beside 520 x 128, which takes two: with 16384 the one took 94 us, the two 10."""
+    from randumb_amd import _lib
+
+    print("case bias gradient of many coefficients", flush=True)
+    lib, k, us = _lib.load(), 16384, []
+    for rows in (512, 520):
+        dy, dc = torch.randn(rows, 128, device="cuda"), torch.empty(k, device="cuda")
+        need = lib.rdb_bias_bwd_workspace_bytes(rows, 128)
+        ws, best = torch.empty(need, dtype=torch.uint8, device="cuda"), 1e9
+        for _ in range(20):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(10):
+                assert lib.rdb_bias_bwd(dc.data_ptr(), 0, dy.data_ptr(), 0, 128, rows, 128, k, 11, ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream) == 0
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end) * 100.0)
+        us.append(best)
+    assert us[0] < us[1] + 30.0, us

@@ -139,12 +139,11 @@ static int dc_room(const rdb_linear_desc *d, int num_cus) { return fg_room(d->ou
 
 // z's ranges that a workspace is asked for: those that pay, whichever products are on (rdb_set_f32_split).  All that z_room allows is up to twice that
 // (2048 x 768, k = 256: 27.3 MB instead of 14.7).
-static double z_host_us(const rdb_linear_desc *d);
 static int z_ranges(const rdb_linear_desc *d, int num_cus)
 {
     const int room = z_room(d, num_cus);
     if (room <= 1 || d->tokens < 32) return room;
-    auto ranges = [&](bool split) { return fg_plan(d->tokens, d->k, d->in_f, num_cus, room, FgGroups<FG_KCONT, FG_NOISE_M>::four, z_host_us(d), split).ranges; };
+    auto ranges = [&](bool split) { return fg_plan(d->tokens, d->k, d->in_f, num_cus, room, FgGroups<FG_KCONT, FG_NOISE_M>::four, 0.0, split).ranges; };
     return std::max(ranges(true), ranges(false));
 }
 static int64_t with_parts(const rdb_linear_desc *d, int ranges) { return up256(d->tokens * d->k * 4) * (ranges > 1 ? 1 + ranges : 1); }
@@ -230,7 +229,8 @@ static int fg_launch_pair_ranges(FgProduct t, int t_room, float *t_part, int64_t
     return fg_launch_sums(sum[0], sum[1], s);
 }
 
-// What z's launch of sums counts for on the host (z_ranges): nothing where the step's products, z, y, t, dC and dx at 1.16 PFLOP/s, take 40 us and more (with as much
+// What z's launch of sums counts for on the host in a training step, which has 60 to 70 us of host work (a forward pass alone has 10, and its kernels are what
+// it waits for: 4700 tokens x 496 -> 32, k = 16 16.2 us a pass, 20.6 with z in one range): nothing where the step's products, z, y, t, dC and dx at 1.16 PFLOP/s, take 40 us and more (with as much
 // again for what they wait, the kernels then outlast the host's 60 to 70: 2859 tokens x 584 -> 7920, k = 208, step 219 us, 222 with z in one range).
 static double z_host_us(const rdb_linear_desc *d)
 {
@@ -240,14 +240,14 @@ static double z_host_us(const rdb_linear_desc *d)
 // z[T x k] = src[T x in_f] . N^T; the partial matrices of its ranges go to `part` (room for max_ranges of them, up256(T k 4)
 // bytes apart; NULL: right behind z, as many as there is room for)
 static int fg_project(float *z, const float *x, int64_t ldx, const rdb_linear_desc *d, int num_cus, hipStream_t s, float *part = nullptr,
-                      int max_ranges = 1 << 30, const FgValues &values = {})
+                      int max_ranges = 1 << 30, double host_us = 0.0, const FgValues &values = {})
 {
     FgProduct q = {x, ldx, (d->tokens - 1) * ldx + d->in_f, nullptr, 0, 0, z, d->k, nullptr, d->tokens, d->k, d->in_f, 0, 0, 0, 0, d->seed};
     q.a_es = fg_es(d->act_dtype);
     q.values = values;
     const int64_t zt = up256(d->tokens * d->k * 4) / 4;
     return fg_launch_ranges<FG_KCONT, FG_NOISE_M>(q, std::max(1, std::min(z_room(d, num_cus), max_ranges)), part ? part : z + zt, zt, num_cus, s,
-                                                  "f32_gemm_kernel (z = x . N^T)", z_host_us(d));
+                                                  "f32_gemm_kernel (z = x . N^T)", host_us);
 }
 
 // Where the forward pass puts the partial matrices of z's ranges: into y, which is written last, or, where y holds less than a third of those that pay, into
@@ -274,7 +274,7 @@ static int fg_project_kept(float *z, const void *x, int64_t ldx, void *y, int64_
     int64_t room = 0;
     if (asked > 0 && scratch_bytes >= asked) part = static_cast<float *>(scratch), room = asked;
     else if (y && ldy == d->out_f && fg_aligned16(y)) part = static_cast<float *>(y), room = d->tokens * d->out_f * fg_es(d->act_dtype);
-    return fg_project(z, static_cast<const float *>(x), ldx, d, num_cus, s, part, (int)std::min<int64_t>(32, room / zt), values);
+    return fg_project(z, static_cast<const float *>(x), ldx, d, num_cus, s, part, (int)std::min<int64_t>(32, room / zt), z_host_us(d), values);
 }
 
 // The three entry points return RDB_E_UNSUPPORTED, without setting an error, when the request does not fit.

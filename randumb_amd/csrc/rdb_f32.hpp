@@ -721,8 +721,16 @@ __device__ __forceinline__ void f32_gemm_block(const FgParams &p, const int bx, 
     }
 }
 
+// Waves a SIMD that registers have to leave room for.  Hashing without a condition per value takes 4 to 8 registers more, which two kinds of tiles do not have
+// to spare: 128 rows of x . R^T, 170 instead of 164 registers, two blocks to a unit instead of three (7028 tokens x 1240 -> 1248 in fp32: 218 us with the
+// condition, 250 without, 208 so), and 64 rows in two groups, 134 instead of 126, one block instead of two.  Asked for, they are found without spills.
+template <int BM, int G, int BSRC> constexpr int fg_min_waves()
+{
+    if (G == 1) return BM == 128 && BSRC == FG_NOISE_1D ? 3 : 2;
+    return G == 2 && BM == 64 && (BSRC == FG_NOISE_M || BSRC == FG_NOISE_I) ? 4 : 1;
+}
 template <int BM, int G, int ASRC, int BSRC, int EPI, bool VEC, bool SPLIT, int AES, int BES>
-__global__ __launch_bounds__(FG_THREADS * G, G == 1 ? 2 : 1) void f32_gemm_kernel(FgParams p)
+__global__ __launch_bounds__(FG_THREADS * G, (fg_min_waves<BM, G, BSRC>())) void f32_gemm_kernel(FgParams p)
 {
     __shared__ __align__(16) float lds[FgBlock<BM, G, ASRC, BSRC, VEC, SPLIT, AES, BES>::LDS];
     __shared__ int not_finite;   // some thread's sum is an infinity or a NaN

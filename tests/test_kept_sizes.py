@@ -43,3 +43,11 @@ def test_nothing_but_what_the_backward_pass_reads(dtype):
             assert 0 <= n <= 33 << 20 and (has or n == 0), (T, in_f, out_f, k, op)
             scratch += n > 0
     assert scratch > 20
+
+
+def test_a_forward_pass_alone_runs_its_projection_in_ranges():
+    """Few tiles of z with long contractions: a training step may do without the launch that adds ranges up, a forward pass waits for its kernels."""
+    lib = _lib.load()
+    for T, in_f, out_f, k in ((4700, 496, 32, 16), (2086, 368, 2352, 8), (470, 336, 3624, 104)):
+        n = lib.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_FWD, ctypes.byref(_desc(T, in_f, out_f, k, _lib.RDB_F32)))
+        assert n >= 3 * _up(4 * T * k), (T, in_f, out_f, k)

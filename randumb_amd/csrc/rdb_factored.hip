@@ -459,18 +459,21 @@ int linear_fwd_projected(void *y, int64_t ldy, const void *state, const void *co
 // scratch of the call's own, 9 MB at most (ranges times tiles are at most the compute units, a sum 32 KB).  With as many ranges as y holds instead: 640
 // tokens x 3400 -> 696, k = 264, one range: 28.6 us, now 20.4; 200 x 8000 -> 1000, k = 400: 39.2, 24.2; 700 x 4000 -> 400, k = 200: 42.6, 26.4; 1056 x
 // 3072 -> 768, k = 240, two ranges: 28.6, 25.5; 2048 x 3072 -> 768, k = 256: 27.8, 24.8.
-constexpr int KZ_MIN_STAGES = 8, KZ_MAX_RANGES = 16;
+// Scratch pays from 22 stages on: two ranges of 8 to 10 stages, which is what shorter inputs get, end 0.5 to 2 us after the one (1024 features: 2303 tokens
+// -> 32, k = 16 15.6 us, in two ranges 16.8; 300 -> 128, k = 256 16.1, 18.2; 3984 -> 152, k = 8 15.9, 17.4; 1536: 19.9, 18.3; 20.4, 18.5; 19.8, 18.2).
+constexpr int KZ_MIN_STAGES = 8, KZ_MAX_RANGES = 16, KZ_SCRATCH_STAGES = 22;
+static int64_t z_part_row(const rdb_linear_desc *d, int64_t ranges);
 static void z_ranges(const rdb_linear_desc *d, int tiles, int &ranges, int &range_stages)
 {
     const int nstage = (int)cdiv(d->in_f, F_BK);
     int64_t r = std::min<int64_t>(std::min<int64_t>(num_compute_units() / tiles, nstage / KZ_MIN_STAGES), KZ_MAX_RANGES);
-    if (r < 1) r = 1;
+    if (r < 1 || (nstage < KZ_SCRATCH_STAGES && z_part_row(d, r) > 0)) r = 1;
     range_stages = (int)cdiv(nstage, r);
     range_stages += range_stages & 1;   // the stages alternate between two buffers, beginning with the first
     ranges = (int)cdiv(nstage, range_stages);
 }
 // bytes of a token's share of the ranges' sums and their tags where y's row does not hold them, else 0
-static int64_t z_part_row(const rdb_linear_desc *d, int ranges)
+static int64_t z_part_row(const rdb_linear_desc *d, int64_t ranges)
 {
     const int64_t kpad = cdiv(d->k, 64) * 64, row = (ranges - 1) * (kpad * 4 + kpad / 4);
     return row + 64 > d->out_f * 2 ? row : 0;

@@ -51,3 +51,10 @@ def test_a_forward_pass_alone_runs_its_projection_in_ranges():
     for T, in_f, out_f, k in ((4700, 496, 32, 16), (2086, 368, 2352, 8), (470, 336, 3624, 104)):
         n = lib.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_FWD, ctypes.byref(_desc(T, in_f, out_f, k, _lib.RDB_F32)))
         assert n >= 3 * _up(4 * T * k), (T, in_f, out_f, k)
+
+
+def test_short_inputs_of_narrow_layers_take_one_range():
+    lib = _lib.load()
+    for in_f, ranges in ((1040, False), (1344, False), (1352, True)):   # 17, 21 and 22 stages of 64 features
+        n = lib.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_PROJECT, ctypes.byref(_desc(2304, in_f, 32, 16, _lib.RDB_BF16)))
+        assert (n > 0) == ranges, (in_f, n)

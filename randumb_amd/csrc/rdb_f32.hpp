@@ -313,7 +313,8 @@ template <int ROWS, int SRC, bool VEC, bool SPLIT = false, int ES = 4> struct Fg
     // apart in the first round).  The main loop calls this between the matrix instructions of the stage before.  Rows and contraction
     // values past the end are hashed as well: such rows' results are not stored, and such contraction values meet zeros of the other
     // side, which is a matrix.  A condition here is a branch around every hash, and no two hashes overlap (1660 tokens x 3902 -> 3361 in
-    // bf16, k = 82, random bias: dy . R 320 -> 287 us, x . R^T 295 -> 263; 616 x 288 -> 1464, k = 40, fp32: z 7.0 -> 6.3).
+    // bf16, k = 82, random bias: dy . R 320 -> 287 us, x . R^T 295 -> 263; 616 x 288 -> 1464, k = 40, fp32: z 7.0 -> 6.3).  Where k is a quarter of a
+    // tile's 128 columns and less, the condition had spared whole waves their hashes, and z is up to 5 % longer (5417 x 1784, k = 10, bf16: 21.7 -> 22.9).
     __device__ __forceinline__ void hash_piece(int stage, int j)
     {
         if constexpr (HASHED) {

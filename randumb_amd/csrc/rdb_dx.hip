@@ -523,7 +523,7 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             // A block of this kernel has a compute unit to itself: where the product's blocks leave units free, no more reduction
             // blocks than those, so that the launch is one round of blocks (8192 tokens x 768 -> 3072, k = 256, 64 units: 9.8 us against
             // 11.2 with 128 blocks).  Less than a quarter of the chip would still be adding long after the product is done, and a second
-            // round is cheaper: 6784 x 576 -> 1728, k = 256, 8 units: 11.6 against 50.4; 4000 x 960 -> 4096, k = 128, 32 units: 8.6
+            // round is cheaper: 6784 x 576 -> 1728, k = 256, 8 units: 10.5 against 50.4; 4000 x 960 -> 4096, k = 128, 32 units: 8.6
             // against 20.0; 8192 x 448 -> 4096, k = 256, 32 units: 11.6 against 18.4.
             const int spare = num_cus - bs.tn_blocks;
             if (spare > 0 && rblocks > spare && std::min(rblocks, num_cus / 2) <= 2 * spare) rblocks = spare;

@@ -231,7 +231,9 @@ static int fg_launch_pair_ranges(FgProduct t, int t_room, float *t_part, int64_t
 
 // What z's launch of sums counts for on the host in a training step, which has 60 to 70 us of host work (a forward pass alone has 10, and its kernels are what
 // it waits for: 4700 tokens x 496 -> 32, k = 16 16.2 us a pass, 20.6 with z in one range): nothing where the step's products, z, y, t, dC and dx at 1.16 PFLOP/s, take 40 us and more (with as much
-// again for what they wait, the kernels then outlast the host's 60 to 70: 2859 tokens x 584 -> 7920, k = 208, step 219 us, 222 with z in one range).
+// again for what they wait, the kernels then outlast the host's 60 to 70: 2859 tokens x 584 -> 7920, k = 208, step 219 us, 222 with z in one range).  Both sides, us a step in six
+// processes each, weighed and not: 207 x 392 -> 1440, k = 56 65.4 to 67.9, 68.1 to 72.5; 181 x 410 -> 3589, k = 293 in bf16 95 to 104, 99 to 104; 1024 x 1024 ->
+// 1024, k = 128 68 to 71 either way.  A process whose host takes 40 a step, one of the twelve, waits for kernels that are 2 to 5 longer instead.
 static double z_host_us(const rdb_linear_desc *d)
 {
     const double parts = d->act_dtype == RDB_BF16 ? 3.0 : 6.0;   // bf16 products per product
@@ -547,7 +549,7 @@ int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, fl
              0, 0, 0, 0, d->seed, (uint32_t)d->in_f, 1u};
         q.dotm = (const float *)dy, q.lddot = lddy;
     }
-    // dx of bf16 layers in as many ranges of the output features as pay and as the workspace, whose t and partial matrices are used up, holds: few
+    // dx of bf16 layers (the kernel that adds the ranges up takes bf16 rows; fp32 layers and the forward share have not been tried in ranges) in as many ranges of the output features as pay and as the workspace, whose t and partial matrices are used up, holds: few
     // tokens are a handful of tiles otherwise, each with all of out_f to hash, split and multiply (us, with the sums: 502 x 527 -> 2918, k = 251: 87 -> 28;
     // 942 x 729 -> 6529, k = 92: 179 -> 59; 1346 x 289 -> 5636, k = 48: 143 -> 38; 1494 x 2739 -> 8065, k = 105: 667 -> 396)
     const int64_t stride = up256(q.M * q.N * 4) / 4, room = (reinterpret_cast<char *>(dots) - static_cast<char *>(workspace)) / (stride * 4);

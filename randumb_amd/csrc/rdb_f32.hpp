@@ -786,7 +786,7 @@ inline FgPlan fg_room(int64_t M, int64_t N, int64_t K, int num_cus, int64_t min_
 // product is short (FG_SHORT_US, and less and less up to FG_LONG_US) ranges have to gain more than both, and 4 % where it
 // is long: a product that fills the chip a little better slows the kernels beside it, which share its power (a vector-coef step of 696 tokens x 856
 // -> 3069, k = 74: y 41.7 -> 39.1 us in three ranges, 3.7 % by the model, the hashing kernels 190 -> 204; dW of 1024 x 768 -> 3072, 4.7 %: 45.5 -> 41.0 and
-// the others as they were).  `resident`, the groups that take turns on a unit's
+// the others as they were: the line lies between these two, no other product near it was measured).  `resident`, the groups that take turns on a unit's
 // time, was fitted with the others and is not what registers and LDS leave room for.  The products measured had fp32 matrices; a
 // side that comes from a bf16 matrix takes less LDS and fewer registers (four to seven blocks of 256 threads fit a unit), and hashing
 // is not told apart: for those the constants are what they are for fp32.

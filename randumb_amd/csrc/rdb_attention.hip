@@ -19,7 +19,7 @@
 // add up at the end.  The longest block is then half as long and there are twice as many, but each stages its tiles for half the
 // rows: for grids that do not keep the compute units busy (at_halves).
 //
-// Measured at 8 sequences x 12 heads x 1024 tokens, us: forward 36.7 (13.5 of them prep), backward 79 (the stock operators they
+// Measured at 8 sequences x 12 heads x 1024 tokens, us: forward 34.7 (13.5 of them prep), backward 79 (the stock operators they
 // replace: attention 81 forward, 267 backward, normalisation and rotation some 450).  13 GFLOP forward and 45 backward.  No pipe is
 // full (SQ counters, shares of a compute unit's time): matrix cores 28 to 30 %, vector ALU 40 to 51 % (29 % of the
 // forward pass in exponentials, 16 a lane for 16 matrix instructions), LDS 36 to 43 % without bank conflicts; two waves a SIMD and a
@@ -187,6 +187,15 @@ __device__ __forceinline__ void at_pack(bf16x8 (&f)[2], const float (&v)[16])
     }
 }
 __device__ __forceinline__ f32x16 at_mma(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+// The loads behind these registers are waited for here.  Operands that a loop only reads: their loads may be scheduled behind those of the
+// first tiles, and loads return in order, so a first use inside the loop waits in every turn for the next tile's loads, which that turn has
+// just requested (forward with preparation, us: 1 x 12 x 1024 21.2 -> 17.5, 4 x 12 x 1024 26.6 -> 24.3, 8 x 12 x 1024 36.7 -> 34.7, 3 x 8 x 200 9.8 ->
+// 9.0; with the tiles requested two steps ahead as well 18.4, 24.1, 36.1, 9.4).
+template <int N> __device__ __forceinline__ void at_arrived(bf16x8 (&f)[N])
+{
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(f[i]));
+}
 // one accumulator (32 x 32) of a wave in LDS, for the other wave of its rows
 __device__ __forceinline__ void at_put(float *lds, const f32x16 &v, int lane)
 {
@@ -252,6 +261,7 @@ template <bool HALVES> __global__ __launch_bounds__(256, 3) void attn_fwd_kernel
     vg.tile(vr, 0);
     at_store_tile(ks_, kr);
     at_store_tile(vs_, vr);
+    at_arrived(qf);
     __syncthreads();
     f32x16 o[2] = {zero16(), zero16()};
     float l = 0.0f;

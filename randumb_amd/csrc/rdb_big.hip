@@ -430,7 +430,7 @@ __global__ __launch_bounds__(256, 1) void big_z_kernel(BigZParams p)
 // The fused random bias's share (rdb_rbias.hip) with R written once as bf16 and read back.  Hashed into the product it costs its hash
 // for every 512 tokens on tiles of 64 features: 75 us for 38.6 GFLOP in either direction at 8192 tokens x 768 -> 3072; here 63 forward
 // (three tiles a block, each with 128 KB of dst to read and write) and 50 backward (one tile of 48 stages a block), and 5 for R.  Tiles
-// of 256 features x 128 tokens, so that 768 features still give 192 of them; one persistent block a compute unit.  What the epilogue
+// of 256 features x 128 tokens, so that 768 features still give 192 of them, or 192 x 128 (rbias_big_rows); one persistent block a compute unit.  What the epilogue
 // adds to is requested before a tile's main loop, the next tile's first stages before its epilogue.
 struct BigRBiasParams {
     const bf16_t *noise;    // [cols x contraction] in fragment order
@@ -444,13 +444,14 @@ struct BigRBiasParams {
 };
 constexpr int BR_TOK = 128;
 
-template <bool DOT> __global__ __launch_bounds__(256, 1) void big_rbias_kernel(BigRBiasParams p)
+template <int BA, bool DOT> __global__ __launch_bounds__(256, 1) void big_rbias_kernel(BigRBiasParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
-    typedef FragOperand<BG, 64> PA;                 // R: rows = columns of dst
+    typedef FragOperand<BA, 64> PA;                 // R: rows = columns of dst
     typedef GlobalOperand<BR_TOK, 64, K_CONT> PB;   // src: rows = tokens
-    constexpr int MI = BG / 64, NI = BR_TOK / 64, LDP = BG / 2 + 4;
+    constexpr int MI = BA / 64, NI = BR_TOK / 64, LDP = BA / 2 + 4;
+    constexpr int LPT = BA / 16, PIECES = 32 * LPT / 64;   // 16-byte pieces of a token's features in a wave's share of the tile; pieces of a lane per 32 tokens
     const int total = p.tiles_a * p.tiles_t, vtotal = (total + 7) / 8 * 8, nblk = gridDim.x, nstage = (p.contraction + 63) / 64;
     int rd = 0;
     auto next = [&]() {
@@ -464,7 +465,7 @@ template <bool DOT> __global__ __launch_bounds__(256, 1) void big_rbias_kernel(B
     PB pb;
     BigRegs<PA, PB> regs;
     auto request = [&](int w) {   // feature tile fastest: neighbours share the tokens
-        frag_rows(pa, p.noise, p.cols, p.contraction, (w % p.tiles_a) * BG);
+        frag_rows(pa, p.noise, p.cols, p.contraction, (w % p.tiles_a) * BA);
         pb = PB{p.src, p.ld_src, (w / p.tiles_a) * BR_TOK, p.tokens, p.contraction, (int64_t)(p.tokens - 1) * p.ld_src + p.contraction};
         big_prefetch(regs, pa, pb, 0);
     };
@@ -480,38 +481,38 @@ template <bool DOT> __global__ __launch_bounds__(256, 1) void big_rbias_kernel(B
     const __amdgpu_buffer_rsrc_t rs_o =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(DOT ? p.other : p.dst), 0, DOT ? (int)(((int64_t)(p.tokens - 1) * p.ld_other + p.cols) * 2) : 0, 0x00020000);
     while (true) {
-        const int a0 = (w % p.tiles_a) * BG, tok0 = (w / p.tiles_a) * BR_TOK;
-        // the thread's pieces of the tile: 8 features of a token; 16 lanes cover a wave's 128 features
+        const int a0 = (w % p.tiles_a) * BA, tok0 = (w / p.tiles_a) * BR_TOK;
+        // the thread's pieces of the tile: 8 features of a token; LPT pieces cover a wave's features
         auto at = [&](int t, int ni, int q, int64_t ld) {
-            const int wave = t >> 6, lane = t & 63, tok = tok0 + (wave & 1) * NI * 32 + ni * 32 + q * 4 + (lane >> 4);
-            const int a = a0 + (wave >> 1) * MI * 32 + (lane & 15) * 8;   // cols is a multiple of 8: a piece lies inside or outside
+            const int wave = t >> 6, e = q * 64 + (t & 63), tok = tok0 + (wave & 1) * NI * 32 + ni * 32 + e / LPT;
+            const int a = a0 + (wave >> 1) * MI * 32 + e % LPT * 8;   // cols is a multiple of 8: a piece lies inside or outside
             return tok < p.tokens && a < p.cols ? (uint32_t)(((int64_t)tok * ld + a) * 2) : BUFFER_OOB;
         };
-        Frag8 old[NI][8];
+        Frag8 old[NI][PIECES];
         {
             const int t = opaque_tid();
 #pragma unroll
             for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
-                for (int q = 0; q < 8; ++q)
+                for (int q = 0; q < PIECES; ++q)
                     old[ni][q].f4 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_d, (int)at(t, ni, q, p.ld_dst), 0, 0));
         }
         f32x16 acc[MI][NI];
-        big_zero<BG, BR_TOK>(acc);
-        big_mainloop<BG, BR_TOK>(acc, lds, regs, pa, pb, nstage);
+        big_zero<BA, BR_TOK>(acc);
+        big_mainloop<BA, BR_TOK>(acc, lds, regs, pa, pb, nstage);
         const int wn = next();
         if (wn >= 0) request(wn);
         __builtin_amdgcn_sched_barrier(0);
         acc_settle<MI, NI>(acc);
         const int t = opaque_tid(), wave = t >> 6, lane = t & 63, r = lane & 31, g = lane >> 5;
-        float *patch = reinterpret_cast<float *>(lds) + wave * 32 * LDP;   // 32 tokens x the wave's 128 features
+        float *patch = reinterpret_cast<float *>(lds) + wave * 32 * LDP;   // 32 tokens x the wave's features
         float dot = 0.0f;
 #pragma unroll
         for (int ni = 0; ni < NI; ++ni) {
-            Frag8 ot[8];
+            Frag8 ot[PIECES];
             if (DOT) {
 #pragma unroll
-                for (int q = 0; q < 8; ++q) ot[q].f4 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_o, (int)at(t, ni, q, p.ld_other), 0, 0));
+                for (int q = 0; q < PIECES; ++q) ot[q].f4 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_o, (int)at(t, ni, q, p.ld_other), 0, 0));
             }
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi)
@@ -522,8 +523,8 @@ template <bool DOT> __global__ __launch_bounds__(256, 1) void big_rbias_kernel(B
             __builtin_amdgcn_sched_barrier(0);
             __builtin_amdgcn_wave_barrier();   // LDS serves a wave's instructions in order: the reads see these writes
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const float *src = patch + (q * 4 + (lane >> 4)) * LDP + (lane & 15) * 8;
+            for (int q = 0; q < PIECES; ++q) {
+                const float *src = patch + (q * 64 + lane) / LPT * LDP + (q * 64 + lane) % LPT * 8;
                 const f32x4 lo = *reinterpret_cast<const f32x4 *>(src), hi = *reinterpret_cast<const f32x4 *>(src + 4);
                 const uint32_t off = at(t, ni, q, p.ld_dst);
                 if (DOT) {   // outside the matrix `ot` reads as zeros
@@ -811,6 +812,18 @@ int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cu
     return bytes;
 }
 
+// Features of a tile of the product above: 192 where as many rounds of tiles as with 256 do, which are more tiles then, for compute units
+// that stood idle.  A round takes 0.93 of one with 256 features (the chip's power again), so another round is never worth it.  us of the step with
+// 256 and with 192 features a tile: 8192 tokens x 768 -> 3072, k = 256, 192 and 256 tiles 179.6, 176.2; 4096 x 1536 -> 4096, k = 128, the same
+// 186.6, 182.4; 8192 x 1024 -> 2048, 256 and 384: 152.9, 166.0; 5000 x 3072 -> 2000, 480 and 640: 222.2, 239.3.
+constexpr int BR_LOW = 192;
+static int rbias_big_rows(int64_t cols, int64_t tokens, int num_cus)
+{
+    auto rounds = [&](int rows) { return cdiv(cdiv(cols, rows) * cdiv(tokens, BR_TOK), num_cus); };
+    return rounds(BR_LOW) <= rounds(BG) ? BR_LOW : BG;
+}
+int64_t rbias_big_tiles(int64_t cols, int64_t tokens, int num_cus) { return cdiv(cols, rbias_big_rows(cols, tokens, num_cus)) * cdiv(tokens, BR_TOK); }
+
 // dst[t, a] += s * sum_c src[t, c] * noise1d(a * sR + c * sK); with `other` also the sum of the product's elements times its, to dscale, with one
 // share per tile in dot_part and a word behind the table.  The caller has checked alignments and extents.
 int linear_rbias_big(void *dst, int64_t ld_dst, int64_t cols, const void *src, int64_t ld_src, int64_t contraction, uint32_t sR, uint32_t sK,
@@ -818,7 +831,8 @@ int linear_rbias_big(void *dst, int64_t ld_dst, int64_t cols, const void *src, i
                      int num_cus, hipStream_t s)
 {
     BigRBiasParams p;
-    p.tiles_a = (int)cdiv(cols, BG);
+    const int ba = rbias_big_rows(cols, d->tokens, num_cus);
+    p.tiles_a = (int)cdiv(cols, ba);
     p.tiles_t = (int)cdiv(d->tokens, BR_TOK);
     const int tiles = p.tiles_a * p.tiles_t;
     p.dscale = {dot_part, other ? reinterpret_cast<unsigned int *>(static_cast<char *>(table) + noise_frag_bytes(cols, contraction)) : nullptr, dscale,
@@ -835,10 +849,14 @@ int linear_rbias_big(void *dst, int64_t ld_dst, int64_t cols, const void *src, i
     p.tokens = (int)d->tokens;
     p.cols = (int)cols;
     p.contraction = (int)contraction;
-    constexpr size_t stages = big_smem<BG, BR_TOK, FragTile<BG, 64>, OperandTile<BR_TOK, 64, K_CONT>>();
-    static_assert((size_t)4 * 32 * (BG / 2 + 4) * sizeof(float) <= stages, "the epilogue's patches fit the pipeline's LDS");
-    if (other) return launch_big(big_rbias_kernel<true>, p, tiles, num_cus, stages, s, "big_rbias_kernel<dot>");
-    return launch_big(big_rbias_kernel<false>, p, tiles, num_cus, stages, s, "big_rbias_kernel");
+    auto run = [&](auto rows, auto dot) {
+        constexpr int BA = decltype(rows)::value;
+        constexpr size_t stages = big_smem<BA, BR_TOK, FragTile<BA, 64>, OperandTile<BR_TOK, 64, K_CONT>>();
+        static_assert((size_t)4 * 32 * (BA / 2 + 4) * sizeof(float) <= stages, "the epilogue's patches fit the pipeline's LDS");
+        return launch_big(big_rbias_kernel<BA, decltype(dot)::value>, p, tiles, num_cus, stages, s, "big_rbias_kernel");
+    };
+    auto with = [&](auto rows) { return other ? run(rows, std::true_type{}) : run(rows, std::false_type{}); };
+    return ba == BG ? with(std::integral_constant<int, BG>{}) : with(std::integral_constant<int, BR_LOW>{});
 }
 
 // y = z . C^T + s * x . R^T (+ bias) from the state, R in `table` (rbias_big_table_bytes of out_f columns)

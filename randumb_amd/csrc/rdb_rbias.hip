@@ -18,6 +18,7 @@ namespace rdb {
 int num_compute_units();   // of the current device (rdb_error.hip)
 // rdb_big.hip
 int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);
+int64_t rbias_big_tiles(int64_t cols, int64_t tokens, int num_cus);
 int linear_rbias_big(void *dst, int64_t ld_dst, int64_t cols, const void *src, int64_t ld_src, int64_t contraction, uint32_t sR, uint32_t sK,
                      const void *scale, const rdb_linear_desc *d, void *table, const void *other, int64_t ld_other, float *dot_part, void *dscale, int dscale_dtype,
                      int num_cus, hipStream_t s);
@@ -540,7 +541,7 @@ static int rbias_add(void *dst, int64_t ld_dst, int64_t cols, const void *src, i
     p.dot_part = dot_part;
     if (other && (ld_other % 8 || ((uintptr_t)other & 15) || d->tokens * ld_other >= (1ll << 29) || !dot_part || !dscale)) return RDB_E_UNSUPPORTED;
     const int64_t need = table ? rbias_big_table_bytes(d, cols, num_compute_units()) : 0;
-    if (need > 0 && table_bytes >= need + (other ? 4 : 0) && !((uintptr_t)table & 15) && (!other || cdiv(cols, 256) * cdiv(d->tokens, 128) <= linear_dx_rbias_dot_floats(d)))
+    if (need > 0 && table_bytes >= need + (other ? 4 : 0) && !((uintptr_t)table & 15) && (!other || rbias_big_tiles(cols, d->tokens, num_compute_units()) <= linear_dx_rbias_dot_floats(d)))
         return linear_rbias_big(dst, ld_dst, cols, src, ld_src, contraction, sR, sK, scale_bias, d, table, other, ld_other, dot_part, dscale, dscale_dtype,
                                 num_compute_units(), s);
     size_t smem = engine_smem<RB_BI, RB_BT, RB_BK, K_CONT, K_CONT>();

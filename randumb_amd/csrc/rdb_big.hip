@@ -698,37 +698,27 @@ int linear_fwd_big(void *y, int64_t ldy, const void *state, const void *coef, co
     return launch_big(big_y_kernel<false>, p, p.tiles_o * p.tiles_t, num_cus, big_smem<BG, BG, TA, TB>(), s, "big_y_kernel");
 }
 
-// The noise as bf16 in fragment order (FragOperand): value (r, c) with first-round value r * row_step + c * col_step + seed, zeros for
-// rows and columns that are padding.  Eight values a thread.  The rounded integers of the kernels that hash into their operands, times
-// 2^-31: a product with either has the same bits.  Fragment order, because a stage of 64 columns then is consecutive kilobytes, not 128
-// bytes of each of 256 rows (4096 tokens x 4096, k = 1024, rows of 8 KB: z 66 -> 62 us; dx, rows of 2 KB: the same).
-__global__ __launch_bounds__(256) void noise_frag_bf16_kernel(bf16_t *__restrict__ out, uint32_t pieces, uint32_t ksteps, uint32_t rows, uint32_t cols,
-                                                              uint32_t row_step, uint32_t col_step, uint32_t seed, unsigned int *cleared)
+// noise_table (rdb_direct.hpp) in a launch of its own, a piece a thread
+__global__ __launch_bounds__(256) void noise_frag_bf16_kernel(NoiseTable table)
 {
-    const uint32_t e = blockIdx.x * 256u + threadIdx.x;
-    if (e == 0 && cleared) *cleared = 0u;   // a word that a later launch counts in
-    if (e >= pieces) return;
-    const uint32_t lane = e & 63u, unit = e >> 6, rb = unit / ksteps, ks = unit - rb * ksteps, r = rb * 32u + (lane & 31u), c = ks * 16u + (lane >> 5) * 8u;
-    i32x4 h = {0, 0, 0, 0};
-    if (r < rows && c < cols) {   // cols is a multiple of 8
-        const uint32_t first = r * row_step + c * col_step + seed;
-        float v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (float)(int32_t)sq5_tail(first + (uint32_t)j * col_step) * 4.656612873077392578125e-10f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) h[j] = (int)f32x2_to_bf16x2(v[2 * j], v[2 * j + 1]);
-    }
-    *reinterpret_cast<i32x4 *>(out + (int64_t)e * 8) = h;
+    noise_table(table, blockIdx.x * 256u + threadIdx.x, gridDim.x * 256u);
 }
 // rows rounded up to 32, columns to 64
 static int64_t noise_frag_bytes(int64_t rows, int64_t cols) { return cdiv(rows, 32) * 32 * cdiv(cols, 64) * 64 * (int64_t)sizeof(bf16_t); }
-static int launch_noise_frag(void *out, int64_t rows, int64_t cols, uint32_t row_step, uint32_t col_step, uint32_t seed, hipStream_t s,
-                             unsigned int *cleared = nullptr)
+static NoiseTable noise_frag_table(void *out, int64_t rows, int64_t cols, uint32_t row_step, uint32_t col_step, uint32_t seed, unsigned int *cleared = nullptr)
 {
-    const uint32_t pieces = (uint32_t)(noise_frag_bytes(rows, cols) / 16);
-    noise_frag_bf16_kernel<<<(unsigned)cdiv(pieces, 256), 256, 0, s>>>(static_cast<bf16_t *>(out), pieces, (uint32_t)(cdiv(cols, 64) * 4), (uint32_t)rows,
-                                                                       (uint32_t)cols, row_step, col_step, seed, cleared);
+    return {static_cast<bf16_t *>(out), (uint32_t)(noise_frag_bytes(rows, cols) / 16), (uint32_t)(cdiv(cols, 64) * 4), (uint32_t)rows, (uint32_t)cols, row_step, col_step,
+            seed, cleared};
+}
+static int launch_noise_frag(const NoiseTable &table, hipStream_t s)
+{
+    noise_frag_bf16_kernel<<<(unsigned)cdiv(table.pieces, 256), 256, 0, s>>>(table);
     return check_launch("noise_frag_bf16_kernel");
+}
+// R [out_f x in_f] of a layer's fused random bias, R[o, i] = noise1d(o * in_f + i)
+NoiseTable rbias_fwd_table(void *out, const rdb_linear_desc *d)
+{
+    return noise_frag_table(out, d->out_f, d->in_f, (uint32_t)d->in_f * SQ5_N1, SQ5_N1, d->seed);
 }
 
 // Scratch for N^T where dx = t . N takes it from memory; 0: where it does not.
@@ -744,7 +734,7 @@ int linear_tn_big(void *dx, int64_t lddx, const void *t, void *table, const rdb_
 {
     if (!dx_big_table_bytes(d, num_cus) || lddx % 8 || d->tokens * lddx >= (1ll << 29) || !big_aligned16(dx) || !big_aligned16(t) || !big_aligned16(table))
         return RDB_E_UNSUPPORTED;
-    if (int rc = launch_noise_frag(table, d->in_f, d->k, PN1, SQ5_N1, d->seed, s)) return rc;   // N^T[i, m] = noise(PRIME * i + m)
+    if (int rc = launch_noise_frag(noise_frag_table(table, d->in_f, d->k, PN1, SQ5_N1, d->seed), s)) return rc;   // N^T[i, m] = noise(PRIME * i + m)
     BigYParams p = {};
     p.zf = static_cast<const bf16_t *>(t);
     p.coef = static_cast<const bf16_t *>(table);
@@ -770,7 +760,7 @@ int linear_z_big(void *state, const void *x, int64_t ldx, const void *coef, void
         return RDB_E_UNSUPPORTED;
     if (ldx % 8 || d->tokens * ldx >= (1ll << 29) || !big_aligned16(x) || !big_aligned16(state) || !big_aligned16(coef) || !big_aligned16(room))
         return RDB_E_UNSUPPORTED;
-    if (int rc = launch_noise_frag(room, d->k, d->in_f, SQ5_N1, PN1, d->seed, s)) return rc;   // N[m, i] = noise(PRIME * i + m)
+    if (int rc = launch_noise_frag(noise_frag_table(room, d->k, d->in_f, SQ5_N1, PN1, d->seed), s)) return rc;   // N[m, i] = noise(PRIME * i + m)
     char *st = static_cast<char *>(state);
     BigZParams p;
     p.noise = static_cast<const bf16_t *>(room);
@@ -837,7 +827,7 @@ int linear_rbias_big(void *dst, int64_t ld_dst, int64_t cols, const void *src, i
     const int tiles = p.tiles_a * p.tiles_t;
     p.dscale = {dot_part, other ? reinterpret_cast<unsigned int *>(static_cast<char *>(table) + noise_frag_bytes(cols, contraction)) : nullptr, dscale,
                 dscale_dtype == RDB_BF16};
-    if (int rc = launch_noise_frag(table, cols, contraction, sR * SQ5_N1, sK * SQ5_N1, d->seed, s, p.dscale.arrived)) return rc;
+    if (int rc = launch_noise_frag(noise_frag_table(table, cols, contraction, sR * SQ5_N1, sK * SQ5_N1, d->seed, p.dscale.arrived), s)) return rc;
     p.noise = static_cast<const bf16_t *>(table);
     p.src = static_cast<const bf16_t *>(src);
     p.dst = static_cast<bf16_t *>(dst);
@@ -859,15 +849,17 @@ int linear_rbias_big(void *dst, int64_t ld_dst, int64_t cols, const void *src, i
     return ba == BG ? with(std::integral_constant<int, BG>{}) : with(std::integral_constant<int, BR_LOW>{});
 }
 
-// y = z . C^T + s * x . R^T (+ bias) from the state, R in `table` (rbias_big_table_bytes of out_f columns)
+// y = z . C^T + s * x . R^T (+ bias) from the state, R in `table` (rbias_big_table_bytes of out_f columns), where it is already if `written`
 int linear_fwd_rbias_big(void *y, int64_t ldy, const void *x, int64_t ldx, const void *state, const void *coef, const void *scale, const void *bias,
-                         const rdb_linear_desc *d, void *table, int num_cus, hipStream_t s)
+                         const rdb_linear_desc *d, void *table, bool written, int num_cus, hipStream_t s)
 {
     const ProjLayout L = proj_layout(d);
     if (!L.ok || d->coef_dtype != RDB_BF16 || ldx % 8 || ldy % 8 || d->tokens * ldx >= (1ll << 29) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     if (!big_aligned16(y) || !big_aligned16(x) || !big_aligned16(state) || !big_aligned16(coef) || !big_aligned16(table) || ((uintptr_t)bias & 7))
         return RDB_E_UNSUPPORTED;
-    if (int rc = launch_noise_frag(table, d->out_f, d->in_f, (uint32_t)d->in_f * SQ5_N1, SQ5_N1, d->seed, s)) return rc;   // R[o, i] = noise1d(o * in_f + i)
+    if (!written) {
+        if (int rc = launch_noise_frag(rbias_fwd_table(table, d), s)) return rc;
+    }
     BigYRParams p;
     p.noise = static_cast<const bf16_t *>(table);
     p.x = static_cast<const bf16_t *>(x);

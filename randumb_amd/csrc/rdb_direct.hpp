@@ -212,4 +212,33 @@ __device__ __forceinline__ void direct_mainloop(f32x16 (&acc)[STAGED_IS_A ? SI :
     RDB_STAMP(2);
 }
 
+// ----------------------------------------------------------------------------------------------- noise written to memory
+// The noise as bf16 in fragment order (FragOperand): value (r, c) with first-round value r * row_step + c * col_step + seed, zeros for
+// rows and columns that are padding.  Eight values a thread and turn.  The rounded integers of the kernels that hash into their operands, times
+// 2^-31: a product with either has the same bits.  Fragment order, because a stage of 64 columns then is consecutive kilobytes, not 128
+// bytes of each of 256 rows (4096 tokens x 4096, k = 1024, rows of 8 KB: z 66 -> 62 us; dx, rows of 2 KB: the same).
+struct NoiseTable {
+    bf16_t *out;
+    uint32_t pieces;          // of 16 bytes; 0: no table
+    uint32_t ksteps, rows, cols, row_step, col_step, seed;
+    unsigned int *cleared;    // NULL, or a word that a later launch counts in
+};
+__device__ __forceinline__ void noise_table(const NoiseTable &p, uint32_t first, uint32_t step)
+{
+    if (first == 0 && p.cleared) *p.cleared = 0u;
+    for (uint32_t e = first; e < p.pieces; e += step) {
+        const uint32_t lane = e & 63u, unit = e >> 6, rb = unit / p.ksteps, ks = unit - rb * p.ksteps, r = rb * 32u + (lane & 31u), c = ks * 16u + (lane >> 5) * 8u;
+        i32x4 h = {0, 0, 0, 0};
+        if (r < p.rows && c < p.cols) {   // cols is a multiple of 8
+            const uint32_t b = r * p.row_step + c * p.col_step + p.seed;
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = (float)(int32_t)sq5_tail(b + (uint32_t)j * p.col_step) * 4.656612873077392578125e-10f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) h[j] = (int)f32x2_to_bf16x2(v[2 * j], v[2 * j + 1]);
+        }
+        *reinterpret_cast<i32x4 *>(p.out + (int64_t)e * 8) = h;
+    }
+}
+
 }  // namespace rdb

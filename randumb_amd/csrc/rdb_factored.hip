@@ -342,11 +342,15 @@ template <bool RANGES> __device__ __forceinline__ void z_block(const ZParams &p,
     RDB_STAMP(3);
 }
 
-template <bool RANGES> __global__ __launch_bounds__(KZ_THREADS, 1) void factored_z_kernel(ZParams p)
+// table: noise that the next launch reads, by the blocks behind those two kinds.  The hash is the vector ALU's, which a projecting block alone does not fill:
+// a launch and most of its time saved (8192 tokens x 768 -> 3072, k = 256, R of the fused random bias: step 172.9 -> 168.1 us).
+template <bool RANGES> __global__ __launch_bounds__(KZ_THREADS, 1) void factored_z_kernel(ZParams p, NoiseTable table)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    if ((int)blockIdx.x < p.z_grid) z_block<RANGES>(p, smem_raw, blockIdx.x, p.z_grid);
-    else transpose_units(p, ((int)blockIdx.x - p.z_grid) * (KZ_THREADS / 64) + (int)(threadIdx.x >> 6), p.c_blocks * (KZ_THREADS / 64));
+    const int block = (int)blockIdx.x - p.z_grid;
+    if (block < 0) z_block<RANGES>(p, smem_raw, blockIdx.x, p.z_grid);
+    else if (block < p.c_blocks) transpose_units(p, block * (KZ_THREADS / 64) + (int)(threadIdx.x >> 6), p.c_blocks * (KZ_THREADS / 64));
+    else noise_table(table, (uint32_t)(block - p.c_blocks) * KZ_THREADS + threadIdx.x, (gridDim.x - (uint32_t)(p.z_grid + p.c_blocks)) * KZ_THREADS);
 }
 
 // ----------------------------------------------------------------------------------------------- y = z . C^T
@@ -565,7 +569,9 @@ static void set_z_grid(ZParams &p, int z_grid, int num_cus)
 static size_t z_smem() { return engine_smem<KZ_BM, KZ_BT, F_BK, K_CONT, K_CONT>(); }
 
 // y: NULL, or the rows of the forward product to come, free to hold sums on the way
-static int launch_z(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, void *scratch, hipStream_t s)
+// table: noise to be written beside it (pieces = 0: none)
+static int launch_z(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, void *scratch, hipStream_t s,
+                    const NoiseTable &table = {})
 {
     ZParams p;
     int rc;
@@ -576,9 +582,9 @@ static int launch_z(void *state, const void *x, int64_t ldx, const void *coef, v
     const void *fn = p.ranges > 1 ? (const void *)factored_z_kernel<true> : (const void *)factored_z_kernel<false>;
     if (int rl = reserve_lds(fn, smem, "factored_z_kernel")) return rl;
     set_z_grid(p, xcd_grid_size(p.tiles_m * p.tiles_t) * (spread ? p.ranges : 1), num_compute_units());
-    const unsigned grid = p.z_grid + p.c_blocks;
-    if (p.ranges > 1) factored_z_kernel<true><<<grid, KZ_THREADS, smem, s>>>(p);
-    else factored_z_kernel<false><<<grid, KZ_THREADS, smem, s>>>(p);
+    const unsigned grid = p.z_grid + p.c_blocks + (unsigned)std::min<int64_t>(cdiv(table.pieces, KZ_THREADS), num_compute_units());
+    if (p.ranges > 1) factored_z_kernel<true><<<grid, KZ_THREADS, smem, s>>>(p, table);
+    else factored_z_kernel<false><<<grid, KZ_THREADS, smem, s>>>(p, table);
     return check_launch("factored_z_kernel");
 }
 
@@ -590,14 +596,17 @@ int linear_project(void *state, const void *x, int64_t ldx, const void *coef, co
 
 // The same ahead of a forward product: y's rows, contiguous and written last, hold N or sums on the way meanwhile.  With a contraction in
 // several ranges the 256-wide tiles' sums would differ from launch_z's (z_ranges).
+// table: NULL, or noise to be written on the way if *written says so afterwards.
 int linear_project_before(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, int num_cus,
-                          hipStream_t s, void *scratch, int64_t scratch_bytes)
+                          hipStream_t s, void *scratch, int64_t scratch_bytes, const NoiseTable *table, bool *written)
 {
     ZParams p;
     if (!fill_z_params(p, state, x, ldx, coef, d)) return RDB_E_UNSUPPORTED;
     const int64_t room = ldy == d->out_f && p.ranges == 1 ? d->tokens * d->out_f * (int64_t)sizeof(bf16_t) : 0;
     const int rc = linear_z_big(state, x, ldx, coef, y, room, d, num_cus, s);
-    return rc != RDB_E_UNSUPPORTED ? rc : launch_z(state, x, ldx, coef, y, ldy, d, enough_scratch(scratch, scratch_bytes, d), s);
+    if (rc != RDB_E_UNSUPPORTED) return rc;
+    if (written) *written = true;
+    return launch_z(state, x, ldx, coef, y, ldy, d, enough_scratch(scratch, scratch_bytes, d), s, table ? *table : NoiseTable{});
 }
 
 // The forward product's parameters when the contraction of a token fits in registers (z in fragment order); returns the
@@ -649,7 +658,7 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
         // check the second call's conditions before the first launch, so that a refusal leaves nothing half done
         if (d->coef_dtype != RDB_BF16 || ldy % 8 || !aligned16(y) || !aligned16(coef)) return RDB_E_UNSUPPORTED;
         if (((uintptr_t)bias & 7) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
-        if (int rc = linear_project_before(state, x, ldx, with_ct ? coef : nullptr, y, ldy, d, num_cus, s, scratch, scratch_bytes)) return rc;
+        if (int rc = linear_project_before(state, x, ldx, with_ct ? coef : nullptr, y, ldy, d, num_cus, s, scratch, scratch_bytes, nullptr, nullptr)) return rc;
         return linear_fwd_projected(y, ldy, state, coef, bias, d, num_cus, s);
     }
     const ProjLayout L = proj_layout(d);

@@ -366,9 +366,10 @@ int linear_dx_rbias_add_dscale(void *dx, int64_t lddx, void *dscale, int dscale_
 int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);
 int64_t rbias_scratch_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);   // rdb_rbias.hip
 int linear_project_before(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, int num_cus,
-                          hipStream_t s, void *scratch, int64_t scratch_bytes);   // rdb_factored.hip
+                          hipStream_t s, void *scratch, int64_t scratch_bytes, const NoiseTable *table, bool *written);   // rdb_factored.hip
 int linear_fwd_rbias_big(void *y, int64_t ldy, const void *x, int64_t ldx, const void *state, const void *coef, const void *scale, const void *bias,
-                         const rdb_linear_desc *d, void *table, int num_cus, hipStream_t s);
+                         const rdb_linear_desc *d, void *table, bool written, int num_cus, hipStream_t s);
+NoiseTable rbias_fwd_table(void *out, const rdb_linear_desc *d);
 
 // rdb_vecsplit.hip
 int64_t linear_vecsplit_workspace(int op, const rdb_linear_desc *d);
@@ -1211,10 +1212,12 @@ extern "C" int rdb_linear_project_fwd_rbias(void *y, int64_t ldy, void *state, c
     hipStream_t s = (hipStream_t)stream;
     int rc = RDB_E_UNSUPPORTED;
     const int64_t table = (project_fwd_rbias_table(d) + 255) / 256 * 256;
+    const NoiseTable noise = rbias_fwd_table(workspace, d);
+    bool written = false;
     if (ldx % 8 == 0 && ldy % 8 == 0 && aligned16(x) && aligned16(y) && aligned16(state) && aligned16(coef) && aligned16(workspace) && !((uintptr_t)bias & 7) &&
         d->tokens * ldx < (1ll << 29) && d->tokens * ldy < (1ll << 29))
-        rc = linear_project_before(state, x, ldx, coef, y, ldy, d, num_compute_units(), s, at_bytes(workspace, table), workspace_bytes - table);
-    if (!rc) rc = linear_fwd_rbias_big(y, ldy, x, ldx, state, coef, scale_bias, bias, d, workspace, num_compute_units(), s);
+        rc = linear_project_before(state, x, ldx, coef, y, ldy, d, num_compute_units(), s, at_bytes(workspace, table), workspace_bytes - table, &noise, &written);
+    if (!rc) rc = linear_fwd_rbias_big(y, ldy, x, ldx, state, coef, scale_bias, bias, d, workspace, written, num_compute_units(), s);
     if (rc == RDB_E_UNSUPPORTED)
         return set_error(rc, "%s: 16-byte aligned pointers (bias: 8-byte), leading dimensions multiples of 8, fewer than 2^29 elements per matrix", who);
     return rc;

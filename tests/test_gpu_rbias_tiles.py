@@ -34,3 +34,22 @@ def test_input_gradient_against_float64(T, in_f, out_f):
     assert float((dx[:, :in_f].double() - want).norm() / want.norm()) < 2e-3   # one rounding to bf16: 2^-9 at most, 1.13e-3 as a norm
     xd = x[:, :in_f].double()
     assert abs(float(ds[0]) - float((dot * xd).sum())) < 1e-5 * float(dot.norm() * xd.norm())   # fp32 sums
+
+
+# R beside a projection in one range of its contraction, in several, and ahead of one on 256-wide tiles (a launch of its own); sizes that are no multiple of
+# a tile, fragment or k-step
+@pytest.mark.parametrize("T,in_f,out_f,k", [(2040, 136, 2056, 8), (2100, 2056, 2008, 72), (8200, 264, 520, 520)])
+def test_forward_against_float64(T, in_f, out_f, k):
+    from randumb_amd import SillyLinear, hip
+
+    print(f"case rbias forward T={T} in={in_f} out={out_f} k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    layer = SillyLinear(in_f, out_f, [k, k], [9, 10], bias=False, rt_bias=True, device="cuda", dtype=torch.bfloat16, matrix_coef=True)
+    with torch.no_grad():
+        layer.weight_coef.normal_(0.0, k**-0.5, generator=g)
+        layer.weight_scale_bias.fill_(0.37)
+    x = torch.randn(T, in_f, device="cuda", generator=g).bfloat16().requires_grad_()
+    y = layer(x)
+    N, R = hip.sq5_fill_2d(in_f, k, 9).double(), hip.sq5_fill_1d(out_f * in_f, 9).view(out_f, in_f).double()
+    want = x.detach().double() @ (layer.weight_coef.detach().double() @ N.t() + layer.weight_scale_bias.detach().double() * R).t()
+    assert float((y.detach().double() - want).norm() / want.norm()) < 6e-3   # N, z, R and y rounded to bf16 once each, 1.13e-3 as a norm; 2^-9 at most

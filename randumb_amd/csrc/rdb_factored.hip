@@ -201,6 +201,31 @@ template <bool RANGES> __device__ __forceinline__ void z_block(const ZParams &p,
         }
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks], fb[ks], acc, 0, 0, 0);
+        // The order the stage is issued in: LDS serves the eight waves' reads and stores one after the other, 100 KB of them, and a wave that has
+        // several to issue waits at the second.  Left to itself the compiler puts all reads and all stores in front and the hash behind
+        // them, in every wave, so LDS and the vector ALU take turns.  A share of the hash between any two of them instead: 8192 tokens x 3072 -> 768,
+        // k = 256, forward 34.9 -> 33.1 us; 768 -> 768 16.9 -> 16.4; 2000 x 4096 -> 4096 30.5 -> 29.9; 1500 x 8192 -> 1024, k = 128, 30.8 -> 29.9.
+        // (The stores first, the reads among the matrix instructions: as before.  Half of the reads of the noise tile, with waves
+        // of 64 tokens that share the k-steps of a stage: no further gain.)
+        if (more) {
+            constexpr int VALU = 0x002, MFMA = 0x008, LOAD = 0x020, LDS_READ = 0x100, LDS_WRITE = 0x200;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                __builtin_amdgcn_sched_group_barrier(VALU, 8, 0);
+                __builtin_amdgcn_sched_group_barrier(LDS_READ, 2, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(VALU, 8, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                __builtin_amdgcn_sched_group_barrier(MFMA, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(LDS_WRITE, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(VALU, 6, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(VALU, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(LDS_WRITE, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(LOAD, XP, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
     for (int rg = my_range; rg < (!RANGES || part ? my_range + 1 : p.ranges); ++rg) {
         int s = RANGES ? rg * p.range_stages : 0;

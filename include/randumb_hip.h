@@ -189,7 +189,7 @@ enum { RDB_OP_LINEAR_FWD = 0, RDB_OP_LINEAR_BWD_DX = 1, RDB_OP_LINEAR_BWD_DCOEF 
        RDB_OP_LINEAR_BWD_PROJECTED_TO = 4, RDB_OP_LINEAR_BWD_DX_DSCALE = 5, RDB_OP_LINEAR_RBIAS_BWD = 6,
        RDB_OP_LINEAR_BWD_KEPT = 7, RDB_OP_LINEAR_RBIAS_FWD = 8,
        RDB_OP_LINEAR_PROJECT_FWD_RBIAS = 9, RDB_OP_LINEAR_RBIAS_BWD_FULL = 10, RDB_OP_LINEAR_PROJECT = 11,
-       RDB_OP_LINEAR_FWD_KEPT = 12 };
+       RDB_OP_LINEAR_FWD_KEPT = 12, RDB_OP_LINEAR_BWD_PROJECTED_RBIAS = 13 };
 
 /* Device scratch (bytes) that entry point `op` can use for `desc`; 0 when it has no use for any.  A NULL or too small
  * workspace is never an error with RDB_ALGO_AUTO: the library then runs a kernel that needs none. */
@@ -380,6 +380,14 @@ int rdb_linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *d
 int rdb_linear_bwd_projected_to(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, const void *dy, int64_t lddy,
                                 const void *state, const void *coef, const rdb_linear_desc *desc, void *workspace,
                                 int64_t workspace_bytes, void *stream);
+
+/* rdb_linear_bwd_projected_to and rdb_linear_rbias_bwd_to in one call, dx = t . N + s * dy . R rounded once: for layers of which
+ * rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_PROJECTED_RBIAS, desc) is not 0, with that many bytes of scratch, 16-byte aligned.
+ * d_scale_bias NULL: the gradient of the scale is not wanted, and x is not read. */
+int rdb_linear_bwd_projected_rbias(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, void *d_scale_bias, int d_scale_bias_dtype,
+                                   const void *dy, int64_t lddy, const void *state, const void *x, int64_t ldx, const void *coef,
+                                   const void *scale_bias, const rdb_linear_desc *desc, void *workspace, int64_t workspace_bytes,
+                                   void *stream);
 
 /* The projected form's counterpart for layers without a projection state (bf16 with sizes that are not multiples of 8, fp32
  * in the few-token regime; rdb_linear_kept_bytes says how much, 0: none, use the calls above): the forward pass leaves

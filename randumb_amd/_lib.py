@@ -20,6 +20,7 @@ RDB_OP_LINEAR_RBIAS_BWD = 6
 RDB_OP_LINEAR_BWD_KEPT = 7
 RDB_OP_LINEAR_PROJECT = 11
 RDB_OP_LINEAR_FWD_KEPT = 12
+RDB_OP_LINEAR_BWD_PROJECTED_RBIAS = 13
 
 # every exported entry point, in header order; tests check the list against the built library
 EXPORTS = [
@@ -49,6 +50,7 @@ EXPORTS = [
     "rdb_linear_rbias_fwd",
     "rdb_linear_rbias_fwd_ws",
     "rdb_linear_project_fwd_rbias",
+    "rdb_linear_bwd_projected_rbias",
     "rdb_linear_rbias_bwd",
     "rdb_linear_rbias_bwd_to",
     "rdb_linear_bwd_dcoef",
@@ -191,6 +193,7 @@ def load() -> ctypes.CDLL:
     L.rdb_linear_bwd_dx_dscale.argtypes = [vp, i64, vp, vp, i64, vp, i64, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_rbias_fwd.argtypes = [vp, i64, vp, i64, vp, dp, vp]
     L.rdb_linear_rbias_fwd_ws.argtypes = [vp, i64, vp, i64, vp, dp, vp, i64, vp]
+    L.rdb_linear_bwd_projected_rbias.argtypes = [vp, i64, vp, ci, vp, ci, vp, i64, vp, vp, i64, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_project_fwd_rbias.argtypes = [vp, i64, vp, i64, vp, vp, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_rbias_bwd.argtypes = [vp, i64, vp, vp, i64, vp, i64, vp, dp, vp, i64, vp]
     L.rdb_linear_rbias_bwd_to.argtypes = [vp, i64, vp, ci, vp, i64, vp, i64, vp, dp, vp, i64, vp]
@@ -239,7 +242,7 @@ def load() -> ctypes.CDLL:
     L.rdb_selftest_hasty_wait.restype = ci
     for name in ("rdb_sq5_fill_2d", "rdb_sq5_fill_1d", "rdb_materialize_fwd", "rdb_materialize_bwd", "rdb_scale_bias_bwd",
                  "rdb_embed_fwd", "rdb_embed_bwd", "rdb_linear_fwd", "rdb_linear_bwd_dx", "rdb_linear_bwd_dx_dscale", "rdb_linear_rbias_fwd",
-                 "rdb_linear_rbias_fwd_ws", "rdb_linear_project_fwd_rbias", "rdb_linear_rbias_bwd", "rdb_linear_rbias_bwd_to", "rdb_linear_bwd_dcoef",
+                 "rdb_linear_rbias_fwd_ws", "rdb_linear_project_fwd_rbias", "rdb_linear_bwd_projected_rbias", "rdb_linear_rbias_bwd", "rdb_linear_rbias_bwd_to", "rdb_linear_bwd_dcoef",
                  "rdb_linear_project", "rdb_linear_project_fwd", "rdb_linear_fwd_projected", "rdb_linear_bwd_dcoef_projected",
                  "rdb_linear_bwd_projected", "rdb_linear_bwd_projected_to", "rdb_linear_bwd_projected_part"):
         getattr(L, name).restype = ci

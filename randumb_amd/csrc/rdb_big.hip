@@ -442,7 +442,7 @@ struct BigRBiasParams {
     int64_t ld_src, ld_dst, ld_other;
     int tokens, cols, contraction, tiles_a, tiles_t;
 };
-constexpr int BR_TOK = 128;
+constexpr int BR_TOK = 128, BR_LOW = 192;   // tokens of a tile; features of the lower kind (rbias_big_rows)
 
 template <int BA, bool DOT> __global__ __launch_bounds__(256, 1) void big_rbias_kernel(BigRBiasParams p)
 {
@@ -634,6 +634,171 @@ template <bool BIAS> __global__ __launch_bounds__(256, 1) void big_yr_kernel(Big
     }
 }
 
+// ----------------------------------------------------------------------------------------------- dx = t . N + s * dy . R
+// The backward pass of a layer with a fused random bias, second launch: a tile contracts dy with R, its sums times x are its share of the scale's
+// gradient; scaled by s they go on with t and N, so that dx is written once, rounded once, and never read back, and N, written down by the launch
+// before like R, is not hashed once a row tile.  Blocks behind the tiles' add up the coefficient gradient's token ranges.  Bound by the matrix cores
+// and the chip's power, like big_rbias_kernel, whose tiles these are; x is read as the accumulators lie, half a cache line a piece, all of it on its
+// way before the main loop.  us of the layer's step with the random bias in launches of its own (the table, dx +=) and with this: 8192 tokens x
+// 768 -> 3072, k = 256: 165.6, 160.2; 4096 x 1536 -> 4096, k = 128: 173.5, 167.3; 8192 x 2048 -> 768, k = 64: 120.7, 111.3; 8192 x 1024 -> 2048,
+// k = 256: 146.8, 138.1; 5000 x 3072 -> 2000, k = 64: 212.1, 202.6; 4096 x 4096 -> 8192, k = 256: 724, 709; no size measured got slower, so all
+// layers take it whose t fits the launch's fragment order (k <= 256) and whose R is written to memory at all (rbias_big_table_bytes).
+struct BigDxParams {
+    const bf16_t *r, *n;    // R [in_f x out_f] and N^T [in_f x k], fragment order
+    const bf16_t *dy;       // [tokens x out_f]
+    const bf16_t *t;        // fragment order, rows = tokens, times 2^-31
+    const bf16_t *scale;    // one value
+    const bf16_t *x;        // DOT: [tokens x in_f]
+    bf16_t *dx;
+    BlockSum dscale;
+    RedParams red;
+    int64_t lddy, ldx, lddx;
+    int tokens, in_f, out_f, k, tiles_a, tiles_t, tile_blocks;
+};
+
+template <int BA, bool DOT> __global__ __launch_bounds__(256, 1) void big_dx_kernel(BigDxParams p)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
+    if ((int)blockIdx.x >= p.tile_blocks) {
+        red_block(p.red, (int)blockIdx.x - p.tile_blocks, (int)gridDim.x - p.tile_blocks);
+        return;
+    }
+    typedef FragOperand<BA, 64> PR;                  // R, and N^T: rows = features
+    typedef GlobalOperand<BR_TOK, 64, K_CONT> PY;    // dy: rows = tokens
+    typedef FragOperand<BR_TOK, 64> PT;              // t: rows = tokens
+    constexpr int MI = BA / 64, NI = BR_TOK / 64, LDP = BA / 2 + 4;
+    constexpr int LPT = BA / 16, PIECES = 32 * LPT / 64;   // as in big_rbias_kernel
+    const int total = p.tiles_a * p.tiles_t, vtotal = (total + 7) / 8 * 8, nblk = p.tile_blocks;
+    int rd = 0;
+    auto next = [&]() {
+        for (; rd * nblk + (int)blockIdx.x < vtotal; ++rd) {
+            const int w = xcd_work_item(rd * nblk + (int)blockIdx.x, total);
+            if (w < total) { ++rd; return w; }
+        }
+        return -1;
+    };
+    PR pr;
+    PY py;
+    BigRegs<PR, PY> regs;
+    auto request = [&](int w) {   // feature tile fastest: neighbours share the tokens
+        frag_rows(pr, p.r, p.in_f, p.out_f, (w % p.tiles_a) * BA);
+        py = PY{p.dy, p.lddy, (w / p.tiles_a) * BR_TOK, p.tokens, p.out_f, (int64_t)(p.tokens - 1) * p.lddy + p.out_f};
+        big_prefetch(regs, pr, py, 0);
+    };
+    auto add_up = [&]() { sum_shares(p.dscale, total, 1, 0, nblk, reinterpret_cast<float *>(lds)); };
+    int w = next();
+    if (w < 0) {   // the grid is rounded up to a multiple of 8: blocks without a tile are counted too
+        if (DOT) add_up();
+        return;
+    }
+    request(w);
+    const float sval = bf16_to_f32(*p.scale);
+    const __amdgpu_buffer_rsrc_t rs_d = __builtin_amdgcn_make_buffer_rsrc(p.dx, 0, (int)(((int64_t)(p.tokens - 1) * p.lddx + p.in_f) * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rs_x =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(DOT ? p.x : p.dx), 0, DOT ? (int)(((int64_t)(p.tokens - 1) * p.ldx + p.in_f) * 2) : 0, 0x00020000);
+    while (true) {
+        const int a0 = (w % p.tiles_a) * BA, tok0 = (w / p.tiles_a) * BR_TOK;
+        PR pn;
+        frag_rows(pn, p.n, p.in_f, p.k, a0);
+        PT pt;
+        frag_rows(pt, p.t, p.tokens, p.k, tok0);
+        BigRegs<PR, PT> regs2;
+        // x as the accumulators lie: four features of a token a lane (in_f is a multiple of 8: all inside or all outside, which reads as zeros)
+        uint2 xv[NI][MI][4];
+        auto load_x = [&](int ni) __attribute__((always_inline)) {
+            const int t = opaque_tid(), wave = t >> 6, lane = t & 63;
+            const int tok = tok0 + (wave & 1) * NI * 32 + ni * 32 + (lane & 31), f = a0 + (wave >> 1) * MI * 32 + 4 * (lane >> 5);
+            const uint32_t at = ((uint32_t)tok * (uint32_t)p.ldx + (uint32_t)f) * 2u;   // a token behind the last is behind the buffer's end too
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+                for (int jq = 0; jq < 4; ++jq) {
+                    const int a = mi * 32 + 8 * jq;
+                    xv[ni][mi][jq] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rs_x, (int)(f + a < p.in_f ? at + 2u * a : BUFFER_OOB), 0, 0));
+                }
+        };
+        // x is requested ahead of the main loop, and what registers still hold: the second contraction's first stage with 192 features or without x
+        constexpr bool BOTH = !DOT || BA == BR_LOW;
+        if (DOT) {
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni) load_x(ni);
+        }
+        if (BOTH) big_prefetch(regs2, pn, pt, 0);
+        f32x16 acc[MI][NI];
+        big_zero<BA, BR_TOK>(acc);
+        big_mainloop<BA, BR_TOK>(acc, lds, regs, pr, py, (p.out_f + 63) / 64);
+        if (!BOTH) big_prefetch(regs2, pn, pt, 0);
+        float dot = 0.0f;
+        acc_settle<MI, NI>(acc);
+        // one accumulator tile at a time, back in its registers and part of the sum before the next is read (see acc_read; with the sum left to the
+        // compiler all values wait for it, 46 of them in scratch)
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) {
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi) {
+#pragma unroll
+                for (int jq = 0; jq < 4; ++jq) {
+                    float v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = acc_read(acc[mi][ni][jq * 4 + e]);
+                    if (DOT) {
+                        const uint2 h = xv[ni][mi][jq];
+                        dot = fmaf(v[0], __uint_as_float(h.x << 16), dot);
+                        dot = fmaf(v[1], __uint_as_float(h.x & 0xffff0000u), dot);
+                        dot = fmaf(v[2], __uint_as_float(h.y << 16), dot);
+                        dot = fmaf(v[3], __uint_as_float(h.y & 0xffff0000u), dot);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[mi][ni][jq * 4 + e] = v[e] * sval;
+                }
+                asm volatile("" : "+a"(acc[mi][ni]), "+v"(dot));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        big_mainloop<BA, BR_TOK>(acc, lds, regs2, pn, pt, (p.k + 63) / 64);
+        const int wn = next();
+        if (wn >= 0) request(wn);
+        __builtin_amdgcn_sched_barrier(0);
+        acc_settle<MI, NI>(acc);
+        const int t = opaque_tid(), wave = t >> 6, lane = t & 63, r = lane & 31, g = lane >> 5;
+        float *patch = reinterpret_cast<float *>(lds) + wave * 32 * LDP;   // 32 tokens x the wave's features
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) {
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+                for (int jq = 0; jq < 4; ++jq)
+                    *reinterpret_cast<f32x4 *>(patch + r * LDP + mi * 32 + 8 * jq + 4 * g) =
+                        f32x4{acc_read(acc[mi][ni][jq * 4]), acc_read(acc[mi][ni][jq * 4 + 1]), acc_read(acc[mi][ni][jq * 4 + 2]), acc_read(acc[mi][ni][jq * 4 + 3])};
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_wave_barrier();   // LDS serves a wave's instructions in order: the reads see these writes
+#pragma unroll
+            for (int q = 0; q < PIECES; ++q) {
+                const int e = q * 64 + lane, tok = tok0 + (wave & 1) * NI * 32 + ni * 32 + e / LPT, a = a0 + (wave >> 1) * MI * 32 + e % LPT * 8;
+                const float *src = patch + e / LPT * LDP + e % LPT * 8;
+                const f32x4 lo = *reinterpret_cast<const f32x4 *>(src), hi = *reinterpret_cast<const f32x4 *>(src + 4);
+                const i32x4 h = {(int)f32x2_to_bf16x2(lo[0], lo[1]), (int)f32x2_to_bf16x2(lo[2], lo[3]), (int)f32x2_to_bf16x2(hi[0], hi[1]), (int)f32x2_to_bf16x2(hi[2], hi[3])};
+                __builtin_amdgcn_raw_buffer_store_b128(h, rs_d, (int)(tok < p.tokens && a < p.in_f ? (uint32_t)(((int64_t)tok * p.lddx + a) * 2) : BUFFER_OOB), 0, 0);
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();   // the patches lie where the next tile's first stage goes
+        if (DOT) {   // lanes, then waves, in a fixed order
+            float *wsum = reinterpret_cast<float *>(lds);
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) dot += __shfl_xor(dot, o, 64);
+            if (lane == 0) wsum[wave] = dot;
+            __syncthreads();
+            if (t == 0) leave_share(p.dscale, w, (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]));
+            __syncthreads();
+        }
+        if (wn < 0) break;
+        w = wn;
+    }
+    if (DOT) add_up();
+}
+
 // ----------------------------------------------------------------------------------------------- host side
 static bool big_aligned16(const void *q) { return ((uintptr_t)q & 15) == 0; }
 
@@ -705,10 +870,11 @@ __global__ __launch_bounds__(256) void noise_frag_bf16_kernel(NoiseTable table)
 }
 // rows rounded up to 32, columns to 64
 static int64_t noise_frag_bytes(int64_t rows, int64_t cols) { return cdiv(rows, 32) * 32 * cdiv(cols, 64) * 64 * (int64_t)sizeof(bf16_t); }
-static NoiseTable noise_frag_table(void *out, int64_t rows, int64_t cols, uint32_t row_step, uint32_t col_step, uint32_t seed, unsigned int *cleared = nullptr)
+static NoiseTable noise_frag_table(void *out, int64_t rows, int64_t cols, uint32_t row_step, uint32_t col_step, uint32_t seed, unsigned int *cleared = nullptr,
+                                   float scale = 4.656612873077392578125e-10f)
 {
     return {static_cast<bf16_t *>(out), (uint32_t)(noise_frag_bytes(rows, cols) / 16), (uint32_t)(cdiv(cols, 64) * 4), (uint32_t)rows, (uint32_t)cols, row_step, col_step,
-            seed, cleared};
+            seed, cleared, scale};
 }
 static int launch_noise_frag(const NoiseTable &table, hipStream_t s)
 {
@@ -720,6 +886,13 @@ NoiseTable rbias_fwd_table(void *out, const rdb_linear_desc *d)
 {
     return noise_frag_table(out, d->out_f, d->in_f, (uint32_t)d->in_f * SQ5_N1, SQ5_N1, d->seed);
 }
+
+// R for dx += s * dy . R, R[i, o] = noise1d(o * in_f + i), and N^T for t . N with a t that has the 2^-31 already
+NoiseTable rbias_dx_table(const RBiasDx &rb, const rdb_linear_desc *d)
+{
+    return noise_frag_table(rb.r, d->in_f, d->out_f, SQ5_N1, (uint32_t)d->in_f * SQ5_N1, d->seed, rb.arrived);
+}
+NoiseTable noise_dx_table(const RBiasDx &rb, const rdb_linear_desc *d) { return noise_frag_table(rb.n, d->in_f, d->k, PN1, SQ5_N1, d->seed, nullptr, 1.0f); }
 
 // Scratch for N^T where dx = t . N takes it from memory; 0: where it does not.
 int64_t dx_big_table_bytes(const rdb_linear_desc *d, int num_cus)
@@ -806,7 +979,6 @@ int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cu
 // that stood idle.  A round takes 0.93 of one with 256 features (the chip's power again), so another round is never worth it.  us of the step with
 // 256 and with 192 features a tile: 8192 tokens x 768 -> 3072, k = 256, 192 and 256 tiles 179.6, 176.2; 4096 x 1536 -> 4096, k = 128, the same
 // 186.6, 182.4; 8192 x 1024 -> 2048, 256 and 384: 152.9, 166.0; 5000 x 3072 -> 2000, 480 and 640: 222.2, 239.3.
-constexpr int BR_LOW = 192;
 static int rbias_big_rows(int64_t cols, int64_t tokens, int num_cus)
 {
     auto rounds = [&](int rows) { return cdiv(cdiv(cols, rows) * cdiv(tokens, BR_TOK), num_cus); };
@@ -881,6 +1053,52 @@ int linear_fwd_rbias_big(void *y, int64_t ldy, const void *x, int64_t ldx, const
     constexpr size_t one = big_smem<BG, BR_TOK, FragTile<BG, 64>, TX>(), two = big_smem<BG, BR_TOK, TC, FragTile<BR_TOK, 64>>(), smem = one > two ? one : two;
     if (bias) return launch_big(big_yr_kernel<true>, p, p.tiles_o * p.tiles_t, num_cus, smem, s, "big_yr_kernel<bias>");
     return launch_big(big_yr_kernel<false>, p, p.tiles_o * p.tiles_t, num_cus, smem, s, "big_yr_kernel");
+}
+
+// dx = t . N + s * dy . R and the scale's gradient, from the tables of rbias_dx_table and noise_dx_table; red: NULL, or sums to be added up beside it
+int linear_dx_rbias_big(void *dx, int64_t lddx, const void *t, const void *dy, int64_t lddy, const RBiasDx &rb, const RedParams *red, const rdb_linear_desc *d,
+                        int num_cus, hipStream_t s)
+{
+    BigDxParams p = {};
+    const int ba = rbias_big_rows(d->in_f, d->tokens, num_cus);
+    p.r = rb.r;
+    p.n = rb.n;
+    p.dy = static_cast<const bf16_t *>(dy);
+    p.t = static_cast<const bf16_t *>(t);
+    p.scale = static_cast<const bf16_t *>(rb.scale);
+    p.x = static_cast<const bf16_t *>(rb.x);
+    p.dx = static_cast<bf16_t *>(dx);
+    p.dscale = {rb.dots, rb.arrived, rb.dscale, rb.dscale_dtype == RDB_BF16};
+    p.lddy = lddy;
+    p.ldx = rb.ldx;
+    p.lddx = lddx;
+    p.tokens = (int)d->tokens;
+    p.in_f = (int)d->in_f;
+    p.out_f = (int)d->out_f;
+    p.k = (int)d->k;
+    p.tiles_a = (int)cdiv(d->in_f, ba);
+    p.tiles_t = (int)cdiv(d->tokens, BR_TOK);
+    const int vtiles = (p.tiles_a * p.tiles_t + 7) / 8 * 8;
+    p.tile_blocks = std::min(std::max(num_cus / 8 * 8, 8), vtiles);
+    int rblocks = 0;
+    if (red) {
+        p.red = *red;
+        rblocks = (int)std::max<int64_t>(1, std::min<int64_t>(cdiv(red->n / 4, 256), num_cus));
+        const int spare = num_cus - p.tile_blocks;
+        if (spare > 0 && rblocks > spare && std::min(rblocks, num_cus / 2) <= 2 * spare) rblocks = spare;   // as beside t . N (linear_bwd_projected)
+    }
+    auto run = [&](auto rows, auto dot) {
+        constexpr int BA = decltype(rows)::value;
+        auto kernel = big_dx_kernel<BA, decltype(dot)::value>;
+        constexpr size_t one = big_smem<BA, BR_TOK, FragTile<BA, 64>, OperandTile<BR_TOK, 64, K_CONT>>();
+        static_assert((size_t)4 * 32 * (BA / 2 + 4) * sizeof(float) <= one && big_smem<BA, BR_TOK, FragTile<BA, 64>, FragTile<BR_TOK, 64>>() <= one,
+                      "the second contraction's stages and the epilogue's patches fit the first one's LDS");
+        if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), one, "big_dx_kernel")) return rl;
+        kernel<<<p.tile_blocks + rblocks, 256, one, s>>>(p);
+        return check_launch("big_dx_kernel");
+    };
+    auto with = [&](auto rows) { return rb.dscale ? run(rows, std::true_type{}) : run(rows, std::false_type{}); };
+    return ba == BG ? with(std::integral_constant<int, BG>{}) : with(std::integral_constant<int, BR_LOW>{});
 }
 
 // First launch of the backward pass: t (row-major, for the t . N kernel of the tile engine) and dC.  `dc`: where the

@@ -125,6 +125,18 @@ struct RedParams {
     int out_bf16;          // 1: out is bf16, the fp32 sum rounded once (not with accumulate)
 };
 
+// What the backward pass of a layer with a fused random bias adds to that of its low-rank share (linear_bwd_projected)
+struct RBiasDx {
+    const void *x;         // with dscale
+    int64_t ldx;
+    const void *scale;     // one bf16 value
+    void *dscale;          // NULL, or where <dy . R, x> goes
+    int dscale_dtype;
+    float *dots;           // one share a tile
+    unsigned int *arrived; // a word
+    bf16_t *r, *n;         // room for R and N^T in fragment order
+};
+
 __device__ __forceinline__ void red_block(const RedParams &p, int block, int nblocks)
 {
     const int64_t n4 = p.n / 4;
@@ -228,6 +240,10 @@ int linear_bwd_big(void *t, void *dc, bool dc_bf16, const void *dy, int64_t lddy
 int linear_z_big(void *state, const void *x, int64_t ldx, const void *coef, void *room, int64_t room_bytes, const rdb_linear_desc *d, int num_cus,
                  hipStream_t s);
 int64_t dx_big_table_bytes(const rdb_linear_desc *d, int num_cus);
+NoiseTable rbias_dx_table(const RBiasDx &rb, const rdb_linear_desc *d);
+NoiseTable noise_dx_table(const RBiasDx &rb, const rdb_linear_desc *d);
+int linear_dx_rbias_big(void *dx, int64_t lddx, const void *t, const void *dy, int64_t lddy, const RBiasDx &rb, const RedParams *red, const rdb_linear_desc *d,
+                        int num_cus, hipStream_t s);
 int linear_tn_big(void *dx, int64_t lddx, const void *t, void *table, const rdb_linear_desc *d, int num_cus, hipStream_t s);
 void set_big_tiles_mode(int mode);
 int big_tiles_mode();

@@ -215,13 +215,14 @@ __device__ __forceinline__ void direct_mainloop(f32x16 (&acc)[STAGED_IS_A ? SI :
 // ----------------------------------------------------------------------------------------------- noise written to memory
 // The noise as bf16 in fragment order (FragOperand): value (r, c) with first-round value r * row_step + c * col_step + seed, zeros for
 // rows and columns that are padding.  Eight values a thread and turn.  The rounded integers of the kernels that hash into their operands, times
-// 2^-31: a product with either has the same bits.  Fragment order, because a stage of 64 columns then is consecutive kilobytes, not 128
+// `scale` (2^-31, or 1 where the other operand has it): a product with either has the same bits.  Fragment order, because a stage of 64 columns then is consecutive kilobytes, not 128
 // bytes of each of 256 rows (4096 tokens x 4096, k = 1024, rows of 8 KB: z 66 -> 62 us; dx, rows of 2 KB: the same).
 struct NoiseTable {
     bf16_t *out;
     uint32_t pieces;          // of 16 bytes; 0: no table
     uint32_t ksteps, rows, cols, row_step, col_step, seed;
     unsigned int *cleared;    // NULL, or a word that a later launch counts in
+    float scale;
 };
 __device__ __forceinline__ void noise_table(const NoiseTable &p, uint32_t first, uint32_t step)
 {
@@ -233,7 +234,7 @@ __device__ __forceinline__ void noise_table(const NoiseTable &p, uint32_t first,
             const uint32_t b = r * p.row_step + c * p.col_step + p.seed;
             float v[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = (float)(int32_t)sq5_tail(b + (uint32_t)j * p.col_step) * 4.656612873077392578125e-10f;
+            for (int j = 0; j < 8; ++j) v[j] = (float)(int32_t)sq5_tail(b + (uint32_t)j * p.col_step) * p.scale;
 #pragma unroll
             for (int j = 0; j < 4; ++j) h[j] = (int)f32x2_to_bf16x2(v[2 * j], v[2 * j + 1]);
         }

@@ -12,6 +12,7 @@
 #include "rdb_blocks.hpp"
 #include "rdb_stationary.hpp"
 #include <algorithm>
+#include <type_traits>
 
 namespace rdb {
 
@@ -256,10 +257,23 @@ struct BwdAParams {
 // fragments, and two stages ahead shorten it (528 tokens x 384 -> 1536, k = 112, 9 blocks of 12 stages: 14.2 us -> 11.7; 700 x 2000 -> 1000, k = 128:
 // 10.0 -> 8.6; 5000 x 1000 -> 1000, k = 64: 10.6 -> 9.4); with a block or more a unit the others' work fills the waits, and the 24 registers are missed
 // (8192 x 768 -> 3072, k = 256: 34.5 -> 36.5; 4096 tokens: 27.7 -> 28.2).
-template <int RD> __global__ __launch_bounds__(256, 2) void bwd_dc_dyc_kernel(BwdAParams p)
+// NOISE: blocks behind those write the two tables that the second launch reads (big_dx_kernel).
+struct BwdTables {
+    NoiseTable r, n;
+    int first;   // their first block
+};
+template <int RD, bool NOISE> __global__ __launch_bounds__(256, 2) void bwd_dc_dyc_kernel(BwdAParams p, std::conditional_t<NOISE, BwdTables, int> tables)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
+    if constexpr (NOISE) {
+        if ((int)blockIdx.x >= tables.first) {
+            const uint32_t at = (blockIdx.x - (uint32_t)tables.first) * 256u + threadIdx.x, step = (gridDim.x - (uint32_t)tables.first) * 256u;
+            noise_table(tables.n, at, step);
+            noise_table(tables.r, at, step);
+            return;
+        }
+    }
     if ((int)blockIdx.x < p.dc_blocks) {
         dc_block_direct(p.dc, lds, blockIdx.x);
     } else {
@@ -440,16 +454,23 @@ int linear_dx_factored(void *dx, int64_t lddx, const void *dy, int64_t lddy, con
 static thread_local int g_bwd_parts = 3;
 void set_bwd_projected_parts(int mask) { g_bwd_parts = mask & 3; }
 
+// Blocks that write the tables, behind the others: short ones, so that every unit that is done with the products finds one.  us of the step with 32,
+// 128, 512 and 1024 of them on 256 units: 8192 tokens x 768 -> 3072, k = 256: 176.4, 167.6, 164.8, 164.4; 4096 x 1536 -> 4096, k = 128: 197.5, 177.1,
+// 169.8, 170.0; 4096 x 4096 -> 8192, k = 256: 856, 727, 707, 717; 8192 x 2048 -> 768, k = 64: 116.8, 113.5, 113.4, 113.5.
+static int table_blocks(uint32_t pieces, int num_cus) { return (int)std::min<int64_t>(cdiv(pieces, 256), 2 * num_cus); }
+
 // Whole backward pass of the layer from the saved projection z: dx = (dy.C).N and dcoef = dy^T.z in two launches.
 // Returns RDB_E_UNSUPPORTED (without setting an error) when the request does not fit.
 // accumulate: dcoef += instead of dcoef = (a later chunk of tokens of a layer whose activations are passed in chunks).
 // dc_bf16: dcoef is bf16 [out_f x k], the fp32 sums rounded once by the blocks that add them up (needs the workspace with room
 // for the sums, linear_bwd_projected_workspace(d, num_cus, true), and is not combined with accumulate).
+// rb: NULL, or the fused random bias's share, for layers whose t stays in registers otherwise (tn_stationary_ok).
 int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, int64_t lddy, const void *z, const void *coef,
                          const rdb_linear_desc *d, int num_cus, void *workspace, int64_t workspace_bytes, bool accumulate, bool dc_bf16,
-                         hipStream_t s)
+                         hipStream_t s, const RBiasDx *rb)
 {
     if (!dx_factored_ok(d)) return RDB_E_UNSUPPORTED;
+    if (rb && (accumulate || !tn_stationary_ok(d, lddx) || workspace_bytes < linear_bwd_projected_workspace(d, num_cus, dc_bf16))) return RDB_E_UNSUPPORTED;
     if (dc_bf16 && (accumulate || workspace_bytes < linear_bwd_projected_workspace(d, num_cus, true))) return RDB_E_UNSUPPORTED;
     if (!workspace || workspace_bytes < linear_dx_factored_workspace(d) || ((uintptr_t)workspace & 15)) return RDB_E_UNSUPPORTED;
     if (d->tokens * lddy >= (1ll << 29) || lddy % 8 || lddx % 8) return RDB_E_UNSUPPORTED;
@@ -491,9 +512,18 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
         } else {
             size_t smem = smem_dc > smem_dyc ? smem_dc : smem_dyc;
             const int dyc_items = p1.tiles_c * p1.tiles_t * (a.dyc.part ? a.dyc.ranges : 1);
-            auto kernel = dyc_items * 2 <= num_cus ? bwd_dc_dyc_kernel<2> : bwd_dc_dyc_kernel<1>;
-            if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem, "bwd_dc_dyc_kernel")) return rl;
-            kernel<<<a.dc_blocks + xcd_grid_size(dyc_items), 256, smem, s>>>(a);
+            const int blocks = a.dc_blocks + xcd_grid_size(dyc_items);
+            if (rb) {
+                const BwdTables tables = {rbias_dx_table(*rb, d), noise_dx_table(*rb, d), blocks};
+                auto kernel = dyc_items * 2 <= num_cus ? bwd_dc_dyc_kernel<2, true> : bwd_dc_dyc_kernel<1, true>;
+                if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem, "bwd_dc_dyc_kernel")) return rl;
+                const int more = table_blocks(tables.r.pieces + tables.n.pieces, num_cus);
+                kernel<<<blocks + more, 256, smem, s>>>(a, tables);
+            } else {
+                auto kernel = dyc_items * 2 <= num_cus ? bwd_dc_dyc_kernel<2, false> : bwd_dc_dyc_kernel<1, false>;
+                if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem, "bwd_dc_dyc_kernel")) return rl;
+                kernel<<<blocks, 256, smem, s>>>(a, 0);
+            }
             rc = check_launch("bwd_dc_dyc_kernel");
             if (!rc && a.dyc.part) {
                 const int k8 = a.dyc.frag_ksteps ? a.dyc.frag_ksteps * 2 : (int)d->k / 8;
@@ -511,6 +541,7 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
         red.splits = red_splits;
         red.accumulate = accumulate ? 1 : 0;
         red.out_bf16 = dc_bf16 ? 1 : 0;
+        if (rb) return linear_dx_rbias_big(dx, lddx, workspace, dy, lddy, *rb, direct ? nullptr : &red, d, num_cus, s);
         if (tn_stationary_ok(d, lddx)) {
             BwdBsParams bs;
             const int items = make_tns_params(bs.tn, dx, lddx, workspace, d, num_cus);

@@ -11,7 +11,7 @@
 // RandumbTensorConstructor.backward -> materialize_bwd / scale_bias_bwd (RandumbTensor.py:979-990).
 #include <algorithm>
 
-#include "rdb_direct.hpp"
+#include "rdb_blocks.hpp"
 #include "rdb_tile.hpp"
 
 namespace rdb {
@@ -338,7 +338,7 @@ int linear_dcoef_f32(float *dcoef, float *d_scale_bias, const void *dy, int64_t 
 // rdb_dx.hip
 int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, int64_t lddy, const void *z, const void *coef,
                          const rdb_linear_desc *d, int num_cus, void *workspace, int64_t workspace_bytes, bool accumulate, bool dc_bf16,
-                         hipStream_t s);
+                         hipStream_t s, const RBiasDx *rb = nullptr);
 int64_t linear_dx_factored_workspace(const rdb_linear_desc *d);
 int64_t linear_bwd_projected_workspace(const rdb_linear_desc *d, int num_cus, bool force_partial);
 int linear_dx_factored(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *coef, const void *scale_bias,
@@ -364,6 +364,7 @@ int linear_dx_rbias_add_dscale(void *dx, int64_t lddx, void *dscale, int dscale_
                                int64_t ldx, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table = nullptr, int64_t table_bytes = 0);
 // rdb_big.hip
 int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);
+int64_t rbias_big_tiles(int64_t cols, int64_t tokens, int num_cus);
 int64_t rbias_scratch_bytes(const rdb_linear_desc *d, int64_t cols, int num_cus);   // rdb_rbias.hip
 int linear_project_before(void *state, const void *x, int64_t ldx, const void *coef, void *y, int64_t ldy, const rdb_linear_desc *d, int num_cus,
                           hipStream_t s, void *scratch, int64_t scratch_bytes, const NoiseTable *table, bool *written);   // rdb_factored.hip
@@ -462,6 +463,10 @@ extern "C" int64_t rdb_linear_workspace_bytes(int op, const rdb_linear_desc *d)
     return need;
 }
 
+struct BwdRBiasRoom {
+    int64_t dots, arrived, r, n, bytes;   // offsets
+};
+static BwdRBiasRoom bwd_projected_rbias_room(const rdb_linear_desc *d);
 static int64_t rbias_dot_room(const rdb_linear_desc *d) { return (linear_dx_rbias_dot_floats(d) * 4 + 255) / 256 * 256; }
 static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d)
 {
@@ -499,6 +504,7 @@ static int64_t linear_workspace_bytes_main(int op, const rdb_linear_desc *d)
         return more > 0 ? rbias_dot_room(d) + more : linear_dx_rbias_dot_floats(d) * 4;   // ... and behind them R, or sums of ranges
     }
     if (op == RDB_OP_LINEAR_PROJECT_FWD_RBIAS) return project_fwd_rbias_bytes(d);
+    if (op == RDB_OP_LINEAR_BWD_PROJECTED_RBIAS) return bwd_projected_rbias_room(d).bytes;
     if (op == RDB_OP_LINEAR_RBIAS_FWD)
         return d->act_dtype == RDB_BF16 && d->coef_dtype == RDB_BF16 ? rbias_scratch_bytes(d, d->out_f, num_compute_units()) : 0;
     if (op == RDB_OP_LINEAR_BWD_PROJECTED || op == RDB_OP_LINEAR_BWD_PROJECTED_TO) {
@@ -1305,6 +1311,53 @@ static int bwd_projected_entry(const char *who, void *dx, int64_t lddx, void *dc
         if (rc) return rc;
     }
     return RDB_OK;
+}
+
+// Workspace of the backward pass of a layer with a fused random bias as two launches: that of the low-rank share, then the tiles' shares of the
+// scale's gradient, a word to count in, R and N^T.  bytes 0: no such form (too few tiles, or a contraction that does not stay in registers).
+static BwdRBiasRoom bwd_projected_rbias_room(const rdb_linear_desc *d)
+{
+    BwdRBiasRoom r = {};
+    const int cus = num_compute_units();
+    if (d->act_dtype != RDB_BF16 || d->coef_dtype != RDB_BF16 || d->coef_rows == 0 || d->sO != d->in_f || d->sI != 1 || d->k > 256 || chunk_plan(d).nchunks != 1) return r;
+    const int64_t table = rbias_big_table_bytes(d, d->in_f, cus), base = rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_PROJECTED_TO, d);
+    if (table <= 0 || base <= 0 || d->tokens * d->in_f >= (1ll << 29) || d->tokens * d->out_f >= (1ll << 29) ||
+        rbias_big_tiles(d->in_f, d->tokens, cus) > linear_dx_rbias_dot_floats(d))
+        return r;
+    auto up = [](int64_t n) { return (n + 255) / 256 * 256; };
+    r.dots = up(base);
+    r.arrived = r.dots + rbias_dot_room(d);
+    r.r = r.arrived + 256;
+    r.n = r.r + up(table);
+    r.bytes = r.n + cdiv(d->in_f, 32) * 32 * cdiv(d->k, 64) * 64 * (int64_t)sizeof(bf16_t);
+    return r;
+}
+
+extern "C" int rdb_linear_bwd_projected_rbias(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, void *d_scale_bias, int d_scale_bias_dtype, const void *dy,
+                                              int64_t lddy, const void *z, const void *x, int64_t ldx, const void *coef, const void *scale_bias,
+                                              const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
+{
+    const char *who = "rdb_linear_bwd_projected_rbias";
+    if (int rc = check_desc(who, d)) return rc;
+    const BwdRBiasRoom room = bwd_projected_rbias_room(d);
+    if (room.bytes <= 0) return set_error(RDB_E_UNSUPPORTED, "%s: a layer that has no such form (rdb_linear_workspace_bytes says 0)", who);
+    if (!dx || !dcoef || !dy || !z || !coef || !scale_bias || (d_scale_bias && !x)) return set_error(RDB_E_NULL, "%s: dx, dcoef, dy, z, x, coef or scale_bias is NULL", who);
+    if (lddx < d->in_f || lddy < d->out_f || (d_scale_bias && ldx < d->in_f)) return set_error(RDB_E_SHAPE, "%s: leading dimension smaller than the row", who);
+    if ((dcoef_dtype != RDB_F32 && dcoef_dtype != RDB_BF16) || (d_scale_bias && d_scale_bias_dtype != RDB_F32 && d_scale_bias_dtype != RDB_BF16))
+        return set_error(RDB_E_DTYPE, "%s: gradients leave as RDB_F32 or RDB_BF16", who);
+    if (!workspace || workspace_bytes < room.bytes) return set_error(RDB_E_WORKSPACE, "%s: needs a workspace of %lld bytes", who, (long long)room.bytes);
+    int rc = RDB_E_UNSUPPORTED;
+    if (lddy % 8 == 0 && lddx % 8 == 0 && aligned16(dy) && aligned16(dx) && aligned16(z) && aligned16(coef) && aligned16(dcoef) && aligned16(workspace) &&
+        d->tokens * lddy < (1ll << 29) && d->tokens * lddx < (1ll << 29) && (!d_scale_bias || (ldx % 8 == 0 && aligned16(x) && d->tokens * ldx < (1ll << 29)))) {
+        const RBiasDx rb = {x, ldx, scale_bias, d_scale_bias, d_scale_bias_dtype, reinterpret_cast<float *>(at_bytes(workspace, room.dots)),
+                            reinterpret_cast<unsigned int *>(at_bytes(workspace, room.arrived)), reinterpret_cast<bf16_t *>(at_bytes(workspace, room.r)),
+                            reinterpret_cast<bf16_t *>(at_bytes(workspace, room.n))};
+        rc = linear_bwd_projected(dx, lddx, static_cast<float *>(dcoef), dy, lddy, z, coef, d, num_compute_units(), workspace, room.dots, false, dcoef_dtype == RDB_BF16,
+                                  (hipStream_t)stream, &rb);
+    }
+    if (rc == RDB_E_UNSUPPORTED)
+        return set_error(rc, "%s: 16-byte aligned pointers, leading dimensions multiples of 8, fewer than 2^29 elements per matrix", who);
+    return rc;
 }
 
 extern "C" int rdb_linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, int64_t lddy, const void *z, const void *coef,

@@ -538,7 +538,19 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         if (c.scalar_type() != dy.scalar_type()) fail(PyExc_RuntimeError, std::string(who) + ": the saved coefficients came back in another dtype");
         restored_values(who, state, dy, at::kByte, rdb_linear_projection_bytes(&d));
         void *s = stream_of(dy);
-        if (want_dc && (want_dx || f32)) {
+        // with the fused random bias: both shares of dx, all gradients, in one call where the layer has such a form (it refuses what the two calls refuse)
+        const int64_t both_shares = has_sb && !f32 && want_dx && want_dc ? rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_PROJECTED_RBIAS, &d) : 0;
+        if (both_shares) {
+            const Tensor x = want_sb ? near_act(saved[3]) : Tensor(), sb = native(scale_bias).to(at::kBFloat16), ws = bytes(both_shares, dy);
+            const auto dt = scale_bias.scalar_type() == at::kBFloat16 ? at::kBFloat16 : at::kFloat;
+            dx = at::empty({dy.size(0), l.in_f}, dy.options());
+            dc = at::empty({c.size(0), c.size(1)}, dy.options().dtype(at::kBFloat16));
+            if (want_sb) dsb = at::empty({1}, dy.options().dtype(dt));
+            check(rdb_linear_bwd_projected_rbias(dx.data_ptr(), l.in_f, dc.data_ptr(), RDB_BF16, ptr(dsb), code(dt), dy.data_ptr(), dy.stride(0), state.data_ptr(),
+                                                 ptr(x), want_sb ? x.stride(0) : 0, c.data_ptr(), sb.data_ptr(), &d, ptr(ws), both_shares, s),
+                  "rdb_linear_bwd_projected_rbias");
+            if (want_sb) dsb = dsb.to(scale_bias.scalar_type());
+        } else if (want_dc && (want_dx || f32)) {
             // bf16 coefficients: their gradient leaves the kernel that adds it up in bf16, where the layer runs as one chunk of tokens
             const bool to_bf16 = !f32 && rdb_linear_projection_chunks(&d, nullptr) == 1;
             const int64_t need = rdb_linear_workspace_bytes(to_bf16 ? RDB_OP_LINEAR_BWD_PROJECTED_TO : RDB_OP_LINEAR_BWD_PROJECTED, &d);
@@ -558,7 +570,7 @@ class ProjectedLinear : public Function<ProjectedLinear> {
             check(rdb_linear_bwd_dcoef_projected(dc.data_ptr<float>(), dy.data_ptr(), dy.stride(0), state.data_ptr(), &d, s), "rdb_linear_bwd_dcoef_projected");
             dc = dc.to(c.scalar_type());
         }
-        if (has_sb && dx.defined()) {
+        if (has_sb && dx.defined() && !both_shares) {
             const Tensor x = near_act(saved[3]), sb = native(scale_bias).to(at::kBFloat16);
             const rdb_linear_desc r = rbias_desc(dy, l);
             const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_BWD_FULL, &r);

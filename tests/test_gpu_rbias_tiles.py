@@ -53,3 +53,49 @@ def test_forward_against_float64(T, in_f, out_f, k):
     N, R = hip.sq5_fill_2d(in_f, k, 9).double(), hip.sq5_fill_1d(out_f * in_f, 9).view(out_f, in_f).double()
     want = x.detach().double() @ (layer.weight_coef.detach().double() @ N.t() + layer.weight_scale_bias.detach().double() * R).t()
     assert float((y.detach().double() - want).norm() / want.norm()) < 6e-3   # N, z, R and y rounded to bf16 once each, 1.13e-3 as a norm; 2^-9 at most
+
+
+# both shares of dx and all gradients in one call: both kinds of tiles, k of one step, of no multiple of a step and the largest; the last case adds up dy . C
+# in ranges.  The scratch holds NaN beforehand; the first case's
+# state has no transposed coefficients
+@pytest.mark.parametrize("T,in_f,out_f,k", [(8100, 584, 72, 8), (5300, 1000, 136, 72), (16385, 200, 264, 200), (16264, 264, 72, 256), (2100, 2056, 2056, 72)])
+def test_backward_in_one_call_against_float64(T, in_f, out_f, k):
+    from randumb_amd import _lib, hip
+
+    print(f"case rbias backward T={T} in={in_f} out={out_f} k={k}", flush=True)
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device="cuda").manual_seed(T)
+    desc = hip._proj_desc(T, in_f, out_f, k, 9)
+    ref = ctypes.byref(desc)
+    n = lib.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_BWD_PROJECTED_RBIAS, ref)
+    assert n >= 2 * in_f * (out_f + k)   # room for R and N
+    C = (torch.randn(out_f, k, device="cuda", generator=g) * k**-0.5).bfloat16()
+    x, dy = (torch.randn(T, cols + 8, device="cuda", generator=g).bfloat16() for cols in (in_f, out_f))
+    s = torch.tensor([0.37], device="cuda").bfloat16()
+    state = hip.linear_project(x[:, :in_f], k, out_f, 9, None if k == 8 else C)
+    ws = torch.full((n + 64,), 0xFF, dtype=torch.uint8, device="cuda")
+
+    def call(dc, ds, room=n):   # ds None: x is not read
+        ws.fill_(0xFF)
+        dx = torch.full((T, in_f + 8), 5.0, device="cuda", dtype=torch.bfloat16)
+        code = {torch.float32: _lib.RDB_F32, torch.bfloat16: _lib.RDB_BF16}
+        rc = lib.rdb_linear_bwd_projected_rbias(dx.data_ptr(), in_f + 8, dc.data_ptr(), code[dc.dtype], None if ds is None else ds.data_ptr(),
+                                                0 if ds is None else code[ds.dtype], dy.data_ptr(), out_f + 8, state.data_ptr(), None if ds is None else x.data_ptr(),
+                                                0 if ds is None else in_f + 8, C.data_ptr(), s.data_ptr(), ref, ws.data_ptr(), room, stream)
+        assert bool((ws[n:] == 0xFF).all()) and bool((dx[:, in_f:] == 5.0).all())
+        return rc, dx[:, :in_f]
+
+    ds, ds16, dc, dc32 = torch.full((2,), 5.0, device="cuda"), torch.full((2,), 5.0, device="cuda").bfloat16(), torch.empty_like(C), C.float()
+    assert call(dc, ds, n - 1)[0] != 0 and float(ds[0]) == 5.0   # refused, not run
+    (rc, dx), (rc16, dx16), (rc32, dx32) = call(dc, ds), call(dc.clone(), ds16), call(dc32, None)
+    assert rc == rc16 == rc32 == 0 and torch.equal(dx, dx16) and torch.equal(dx, dx32)
+    assert float(ds[1]) == float(ds16[1]) == 5.0 and torch.equal(ds[:1].bfloat16(), ds16[:1])
+    # the coefficients' gradient is that of the layer without the bias, to the bit
+    for got in (dc, dc32):
+        want = hip.linear_bwd_projected(dy[:, :out_f], state, C, in_f, 9, dcoef_dtype=got.dtype)[1]
+        assert torch.equal(got, want)
+    N, R, xd, dyd = hip.sq5_fill_2d(in_f, k, 9).double(), hip.sq5_fill_1d(out_f * in_f, 9).view(out_f, in_f).double(), x[:, :in_f].double(), dy[:, :out_f].double()
+    dot = dyd @ R.bfloat16().double()
+    want = dyd @ C.double() @ N.t() + s.double() * dyd @ R
+    assert float((dx.double() - want).norm() / want.norm()) < 6e-3   # N, t, R and dx rounded to bf16 once each, 1.13e-3 as a norm; 2^-9 at most
+    assert abs(float(ds[0]) - float((dot * xd).sum())) < 1e-5 * float(dot.norm() * xd.norm())   # fp32 sums

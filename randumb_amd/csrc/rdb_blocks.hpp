@@ -134,7 +134,7 @@ struct RBiasDx {
     int dscale_dtype;
     float *dots;           // one share a tile
     unsigned int *arrived; // a word
-    bf16_t *r, *n;         // room for R and N^T in fragment order
+    bf16_t *r, *n;         // room for R and N^T in fragment order (without a random bias: n alone)
 };
 
 __device__ __forceinline__ void red_block(const RedParams &p, int block, int nblocks)

@@ -257,7 +257,7 @@ struct BwdAParams {
 // fragments, and two stages ahead shorten it (528 tokens x 384 -> 1536, k = 112, 9 blocks of 12 stages: 14.2 us -> 11.7; 700 x 2000 -> 1000, k = 128:
 // 10.0 -> 8.6; 5000 x 1000 -> 1000, k = 64: 10.6 -> 9.4); with a block or more a unit the others' work fills the waits, and the 24 registers are missed
 // (8192 x 768 -> 3072, k = 256: 34.5 -> 36.5; 4096 tokens: 27.7 -> 28.2).
-// NOISE: blocks behind those write the two tables that the second launch reads (big_dx_kernel).
+// NOISE: blocks behind those write the tables that the second launch reads: N, and with a fused random bias R (big_dx_kernel).
 struct BwdTables {
     NoiseTable r, n;
     int first;   // their first block
@@ -312,11 +312,11 @@ struct BwdBsParams {
     int tn_blocks;
 };
 
-template <int KG, int AUX> __global__ __launch_bounds__(ST_THREADS, 1) void bwd_tns_red_kernel(BwdBsParams p)
+template <int KG, int AUX, bool TABLE> __global__ __launch_bounds__(ST_THREADS, 1) void bwd_tns_red_kernel(BwdBsParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     if ((int)blockIdx.x < p.tn_blocks)
-        stationary_block<KG, false, true, AUX, true>(p.tn, smem_raw, blockIdx.x);
+        stationary_block<KG, false, !TABLE, AUX, true, TABLE>(p.tn, smem_raw, blockIdx.x);
     else
         red_block(p.red, blockIdx.x - p.tn_blocks, gridDim.x - p.tn_blocks);
 }
@@ -392,13 +392,30 @@ static void make_dyc_params(DyCParams &p1, const void *dy, int64_t lddy, const v
     p1.frag_ksteps = 0;
 }
 
-// Scratch of the regrouped backward pass that it can do without: the ranges' sums, and later, in their place, N^T for dx = t . N
+// Scratch for N^T where dx = t . N with t in registers takes it from memory, written by the first launch beside its products; 0: where it is hashed
+// under the matrix instructions.  Those hide the hash of a unit of up to 128 coefficients, no more: from 136 up each step of a block is the vector
+// ALU's.  Not where a block takes one unit (nothing is hashed under anything, and the units come from memory a round trip later), nor below 12 token
+// tiles (every value is hashed once a tile), nor with two units where adding up a large dC beside them takes as long.  us of the backward call,
+// hashed and from memory: 8192 tokens x 3072 -> 768, k = 256, 192, 128 and 64: 44.9, 37.5; 40.0, 36.5; 35.6, 36.1; 27.6, 29.7; 8192 x 768 -> 768,
+// k = 256 (two units): 24.9, 24.4; 3072 x 8192 -> 1024, k = 136: 45.5, 36.0; 6000 x 1000 -> 1000, k = 192: 25.3, 23.5; 3072 x 3072 -> 4096, k = 256:
+// 39.3, 39.6; one unit: 4096 x 768 -> 768, k = 256: 20.6, 21.2; two and a large dC: 8192 x 768 -> 3072, k = 256: 42.6, 43.0; 9 tiles: 2304 x 3072 ->
+// 768, k = 256: 20.0, 20.5; 3 tiles: 600 x 4096 -> 512, k = 256: 12.5, 13.7.
+static int64_t tns_table_bytes(const rdb_linear_desc *d, int num_cus)
+{
+    const int64_t bytes = cdiv(d->in_f, 32) * 32 * cdiv(d->k, 64) * 64 * (int64_t)sizeof(bf16_t);
+    if (d->k <= 128 || d->k > ST_KMAX || bytes >= (1ll << 30)) return 0;
+    StParams q;
+    make_stationary_grid(q, d->tokens, d->in_f, num_cus);
+    return q.tiles_t >= 12 && q.units_per_split >= (d->out_f <= 2 * d->in_f ? 2 : 3) ? bytes : 0;
+}
+// Scratch of the regrouped backward pass that it can do without: the ranges' sums and behind them, or later in their place (k > 256), N^T for dx = t . N
 int64_t linear_bwd_projected_extra(const rdb_linear_desc *d, int num_cus)
 {
     if (!dx_factored_ok(d)) return 0;
     int len;
     const int ranges = dyc_ranges(d, num_cus, &len);
-    return std::max<int64_t>(ranges > 1 ? align256(ranges * d->tokens * d->k * (int64_t)sizeof(float)) : 0, dx_big_table_bytes(d, num_cus));
+    const int64_t part = ranges > 1 ? align256(ranges * d->tokens * d->k * (int64_t)sizeof(float)) : 0;
+    return std::max<int64_t>(part + tns_table_bytes(d, num_cus), dx_big_table_bytes(d, num_cus));
 }
 
 // t . N with t in registers applies when k is short enough and dx fits a buffer descriptor.
@@ -501,6 +518,10 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
         const int64_t base = align256(linear_bwd_projected_workspace(d, num_cus, accumulate || dc_bf16));
         if (a.dyc.ranges > 1 && workspace_bytes >= base + align256(a.dyc.ranges * d->tokens * d->k * (int64_t)sizeof(float)))
             a.dyc.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + base);
+        const int64_t table_at = base + (a.dyc.part ? align256(a.dyc.ranges * d->tokens * d->k * (int64_t)sizeof(float)) : 0), table_n = tns_table_bytes(d, num_cus);
+        RBiasDx nt = {};
+        if (!rb && table_n && tn_stationary_ok(d, lddx) && workspace_bytes >= table_at + table_n)
+            nt.n = reinterpret_cast<bf16_t *>(static_cast<char *>(workspace) + table_at);
         a.dc_blocks = xcd_grid_size(dc_items);
         int rc = RDB_OK;
         const int red_splits = big ? 1 : a.dc.splits;
@@ -513,12 +534,11 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             size_t smem = smem_dc > smem_dyc ? smem_dc : smem_dyc;
             const int dyc_items = p1.tiles_c * p1.tiles_t * (a.dyc.part ? a.dyc.ranges : 1);
             const int blocks = a.dc_blocks + xcd_grid_size(dyc_items);
-            if (rb) {
-                const BwdTables tables = {rbias_dx_table(*rb, d), noise_dx_table(*rb, d), blocks};
+            if (rb || nt.n) {
+                const BwdTables tables = {rb ? rbias_dx_table(*rb, d) : NoiseTable{}, noise_dx_table(rb ? *rb : nt, d), blocks};
                 auto kernel = dyc_items * 2 <= num_cus ? bwd_dc_dyc_kernel<2, true> : bwd_dc_dyc_kernel<1, true>;
                 if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem, "bwd_dc_dyc_kernel")) return rl;
-                const int more = table_blocks(tables.r.pieces + tables.n.pieces, num_cus);
-                kernel<<<blocks + more, 256, smem, s>>>(a, tables);
+                kernel<<<blocks + table_blocks(tables.r.pieces + tables.n.pieces, num_cus), 256, smem, s>>>(a, tables);
             } else {
                 auto kernel = dyc_items * 2 <= num_cus ? bwd_dc_dyc_kernel<2, false> : bwd_dc_dyc_kernel<1, false>;
                 if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem, "bwd_dc_dyc_kernel")) return rl;
@@ -560,8 +580,10 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             if (spare > 0 && rblocks > spare && std::min(rblocks, num_cus / 2) <= 2 * spare) rblocks = spare;
             if (rblocks < 1) rblocks = 1;
             if (direct) rblocks = 0;
+            bs.tn.coef = nt.n;
             return with_stationary_variant(bs.tn, [&](auto kg, auto aux) {
-                auto kernel = bwd_tns_red_kernel<decltype(kg)::value, decltype(aux)::value>;
+                constexpr int KG = decltype(kg)::value, AUX = decltype(aux)::value;
+                auto kernel = nt.n ? bwd_tns_red_kernel<KG, AUX, (KG > 2)> : bwd_tns_red_kernel<KG, AUX, false>;   // no table up to k = 128
                 const size_t smem_s = stationary_smem(kg);
                 if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem_s, "bwd_tns_red_kernel")) return rl;
                 kernel<<<bs.tn_blocks + rblocks, ST_THREADS, smem_s, s>>>(bs);

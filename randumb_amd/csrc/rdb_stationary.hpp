@@ -29,7 +29,7 @@ constexpr int ST_KMAX = 256;
 struct StParams {
     const bf16_t *z;     // left operand [tokens x k]: row-major, or (ZFRAG) in fragment order as store_tile_bf16_frag writes it,
                          // tokens padded to 32 and k to KG * 64, the noise flavour's 2^-31 already applied
-    const bf16_t *coef;  // right operand [out_f x k] (not used when the right operand is noise)
+    const bf16_t *coef;  // right operand [out_f x k], or (TABLE) in fragment order; not used when the right operand is noise
     const bf16_t *bias;  // [out_f] or NULL
     bf16_t *y;           // [tokens x out_f], leading dimension ldy
     int64_t ldy;
@@ -48,7 +48,8 @@ struct StParams {
 // rows are 2^31 * noise(PRIME*row + m), hashed into the tile; the producer of the left operand has scaled it by 2^-31
 // (exact in bf16).  AUX: cache policy of the row stores (an immediate of the instruction: two copies of the steps in one kernel cost it 10 to 20
 // registers, and spills with k = 256 and a bias).
-template <int KG, bool BIAS, bool NOISE, int AUX> struct StBlock {
+// TABLE: `coef` is in fragment order (rows padded to 32, k to kpad, zeros there): a unit's tile is consecutive kilobytes.
+template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE> struct StBlock {
     static constexpr int kpad = KG * 64, ldk = kpad + 8, cpr = kpad / 8, ncp = ST_BO * cpr, NQ = ncp / ST_THREADS;
     const StParams &p;
     bf16_t *Cs;   // [2][64 rows][ldk]
@@ -64,6 +65,12 @@ template <int KG, bool BIAS, bool NOISE, int AUX> struct StBlock {
 
     __device__ __forceinline__ void issue(int unit)
     {   // global -> registers for a C tile; rows past out_f read as zeros
+        if constexpr (TABLE) {
+            const uint32_t at = (uint32_t)(unit * ncp + t) * 16u;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) rc[q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_c, (int)(at + (uint32_t)(q * ST_THREADS * 16)), 0, 0));
+            return;
+        }
         const int o0 = unit * ST_BO, left = p.out_f - o0;
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
@@ -94,7 +101,12 @@ template <int KG, bool BIAS, bool NOISE, int AUX> struct StBlock {
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
             const int idx = q * ST_THREADS + t;
-            *reinterpret_cast<f32x4 *>(cn + (idx / cpr) * ldk + (idx % cpr) * 8) = rc[q];
+            if constexpr (TABLE) {   // 64 pieces a k-step, of 32 rows
+                constexpr int half = ncp / 2;
+                *reinterpret_cast<f32x4 *>(cn + (idx / half * 32 + (idx & 31)) * ldk + idx % half / 64 * 16 + ((idx >> 5) & 1) * 8) = rc[q];
+            } else {
+                *reinterpret_cast<f32x4 *>(cn + (idx / cpr) * ldk + (idx % cpr) * 8) = rc[q];
+            }
         }
     }
 
@@ -201,10 +213,10 @@ template <int KG, bool BIAS, bool NOISE, int AUX> struct StBlock {
 };
 
 // `block`: index of this block among the blocks that run this body; all ST_THREADS threads of the block must call.
-template <int KG, bool BIAS, bool NOISE, int AUX, bool ZFRAG = false>
+template <int KG, bool BIAS, bool NOISE, int AUX, bool ZFRAG = false, bool TABLE = false>
 __device__ __forceinline__ void stationary_block(const StParams &p, unsigned char *smem_raw, int block)
 {
-    typedef StBlock<KG, BIAS, NOISE, AUX> B;
+    typedef StBlock<KG, BIAS, NOISE, AUX, TABLE> B;
     const int t = threadIdx.x, wave = t >> 6;
     // work item = (token tile, split), split fastest: neighbours share the left operand's tile, everyone shares the right operand
     const int w = xcd_work_item(block, p.tiles_t * p.splits);
@@ -220,7 +232,8 @@ __device__ __forceinline__ void stationary_block(const StParams &p, unsigned cha
     b.nunits = min(p.units_per_split, (p.out_f + ST_BO - 1) / ST_BO - b.unit0);
     if (b.nunits <= 0) return;
     RDB_STAMP(0);
-    b.rs_c = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(p.coef), 0, NOISE ? 0 : (int)((int64_t)p.out_f * p.k * 2), 0x00020000);
+    b.rs_c = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(p.coef), 0,
+                                               NOISE ? 0 : TABLE ? (p.out_f + 31) / 32 * 32 * B::kpad * 2 : (int)((int64_t)p.out_f * p.k * 2), 0x00020000);
     b.rs_y = __builtin_amdgcn_make_buffer_rsrc(p.y, 0, (int)(((int64_t)(p.tokens - 1) * p.ldy + p.out_f) * 2), 0x00020000);
     b.rs_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(p.bias), 0, p.bias ? p.out_f * 2 : 0, 0x00020000);  // no bias: zeros
     b.t = t;

@@ -142,7 +142,7 @@ template <bool BIAS, bool FRAG = true> __global__ __launch_bounds__(256, 1) void
             if (wn >= 0) request(wn);   // on its way while this tile leaves
             __builtin_amdgcn_sched_barrier(0);
             RDB_STAMP(2);
-            big_store_bf16<BG, BG, BIAS, STORE_STREAM>(acc, lds, p.y, p.ldy, p.y_elems, o0, p.out_f, tok0, p.tokens, bias, opaque_tid());
+            big_store_bf16<BG, BG, BIAS, true>(acc, lds, p.y, p.ldy, p.y_elems, o0, p.out_f, tok0, p.tokens, bias, opaque_tid());
             RDB_STAMP(3);
 #ifdef RDB_STAMPS
             ++rdb_stamp_seq;
@@ -171,7 +171,7 @@ template <bool BIAS, bool FRAG = true> __global__ __launch_bounds__(256, 1) void
         BigBias<BG> bias;
         if (BIAS) big_load_bias<BG>(bias, p.bias, o0, p.out_f);
         RDB_STAMP(2);
-        big_store_bf16<BG, BY_HALF, BIAS, STORE_STREAM>(acc, lds, p.y, p.ldy, p.y_elems, o0, p.out_f, tok0, p.tokens, bias, opaque_tid());
+        big_store_bf16<BG, BY_HALF, BIAS, true>(acc, lds, p.y, p.ldy, p.y_elems, o0, p.out_f, tok0, p.tokens, bias, opaque_tid());
         RDB_STAMP(3);
     }
 }
@@ -578,7 +578,7 @@ struct BigYRParams {
     int tokens, in_f, out_f, k, tiles_o, tiles_t;
 };
 
-template <bool BIAS, int AUX> __global__ __launch_bounds__(256, 1) void big_yr_kernel(BigYRParams p)
+template <bool BIAS> __global__ __launch_bounds__(256, 1) void big_yr_kernel(BigYRParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
@@ -628,7 +628,7 @@ template <bool BIAS, int AUX> __global__ __launch_bounds__(256, 1) void big_yr_k
         const int wn = next();
         if (wn >= 0) request(wn);
         __builtin_amdgcn_sched_barrier(0);
-        big_store_bf16<BG, BR_TOK, BIAS, AUX>(acc, lds, p.y, p.ldy, (int64_t)(p.tokens - 1) * p.ldy + p.out_f, o0, p.out_f, tok0, p.tokens, bias, opaque_tid());
+        big_store_bf16<BG, BR_TOK, BIAS, true>(acc, lds, p.y, p.ldy, (int64_t)(p.tokens - 1) * p.ldy + p.out_f, o0, p.out_f, tok0, p.tokens, bias, opaque_tid());
         if (wn < 0) break;
         w = wn;
     }
@@ -656,7 +656,7 @@ struct BigDxParams {
     int tokens, in_f, out_f, k, tiles_a, tiles_t, tile_blocks;
 };
 
-template <int BA, bool DOT, int AUX> __global__ __launch_bounds__(256, 1) void big_dx_kernel(BigDxParams p)
+template <int BA, bool DOT> __global__ __launch_bounds__(256, 1) void big_dx_kernel(BigDxParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);
@@ -779,7 +779,7 @@ template <int BA, bool DOT, int AUX> __global__ __launch_bounds__(256, 1) void b
                 const float *src = patch + e / LPT * LDP + e % LPT * 8;
                 const f32x4 lo = *reinterpret_cast<const f32x4 *>(src), hi = *reinterpret_cast<const f32x4 *>(src + 4);
                 const i32x4 h = {(int)f32x2_to_bf16x2(lo[0], lo[1]), (int)f32x2_to_bf16x2(lo[2], lo[3]), (int)f32x2_to_bf16x2(hi[0], hi[1]), (int)f32x2_to_bf16x2(hi[2], hi[3])};
-                __builtin_amdgcn_raw_buffer_store_b128(h, rs_d, (int)(tok < p.tokens && a < p.in_f ? (uint32_t)(((int64_t)tok * p.lddx + a) * 2) : BUFFER_OOB), 0, AUX);
+                __builtin_amdgcn_raw_buffer_store_b128(h, rs_d, (int)(tok < p.tokens && a < p.in_f ? (uint32_t)(((int64_t)tok * p.lddx + a) * 2) : BUFFER_OOB), 0, 0);
             }
             __builtin_amdgcn_wave_barrier();
         }
@@ -1051,12 +1051,8 @@ int linear_fwd_rbias_big(void *y, int64_t ldy, const void *x, int64_t ldx, const
     typedef OperandTile<BG, 64, K_CONT> TC;
     typedef OperandTile<BR_TOK, 64, K_CONT> TX;
     constexpr size_t one = big_smem<BG, BR_TOK, FragTile<BG, 64>, TX>(), two = big_smem<BG, BR_TOK, TC, FragTile<BR_TOK, 64>>(), smem = one > two ? one : two;
-    auto run = [&](auto aux) {
-        constexpr int AUX = decltype(aux)::value;
-        if (bias) return launch_big(big_yr_kernel<true, AUX>, p, p.tiles_o * p.tiles_t, num_cus, smem, s, "big_yr_kernel<bias>");
-        return launch_big(big_yr_kernel<false, AUX>, p, p.tiles_o * p.tiles_t, num_cus, smem, s, "big_yr_kernel");
-    };
-    return with_store_policy(y, ldy, d->tokens * (d->in_f + d->out_f) * 2, run);
+    if (bias) return launch_big(big_yr_kernel<true>, p, p.tiles_o * p.tiles_t, num_cus, smem, s, "big_yr_kernel<bias>");
+    return launch_big(big_yr_kernel<false>, p, p.tiles_o * p.tiles_t, num_cus, smem, s, "big_yr_kernel");
 }
 
 // dx = t . N + s * dy . R and the scale's gradient, from the tables of rbias_dx_table and noise_dx_table; red: NULL, or sums to be added up beside it
@@ -1091,9 +1087,9 @@ int linear_dx_rbias_big(void *dx, int64_t lddx, const void *t, const void *dy, i
         const int spare = num_cus - p.tile_blocks;
         if (spare > 0 && rblocks > spare && std::min(rblocks, num_cus / 2) <= 2 * spare) rblocks = spare;   // as beside t . N (linear_bwd_projected)
     }
-    auto run = [&](auto rows, auto dot, auto aux) {
+    auto run = [&](auto rows, auto dot) {
         constexpr int BA = decltype(rows)::value;
-        auto kernel = big_dx_kernel<BA, decltype(dot)::value, decltype(aux)::value>;
+        auto kernel = big_dx_kernel<BA, decltype(dot)::value>;
         constexpr size_t one = big_smem<BA, BR_TOK, FragTile<BA, 64>, OperandTile<BR_TOK, 64, K_CONT>>();
         static_assert((size_t)4 * 32 * (BA / 2 + 4) * sizeof(float) <= one && big_smem<BA, BR_TOK, FragTile<BA, 64>, FragTile<BR_TOK, 64>>() <= one,
                       "the second contraction's stages and the epilogue's patches fit the first one's LDS");
@@ -1101,10 +1097,8 @@ int linear_dx_rbias_big(void *dx, int64_t lddx, const void *t, const void *dy, i
         kernel<<<p.tile_blocks + rblocks, 256, one, s>>>(p);
         return check_launch("big_dx_kernel");
     };
-    return with_store_policy(dx, lddx, d->tokens * (d->in_f + d->out_f) * 2, [&](auto aux) {
-        auto with = [&](auto rows) { return rb.dscale ? run(rows, std::true_type{}, aux) : run(rows, std::false_type{}, aux); };
-        return ba == BG ? with(std::integral_constant<int, BG>{}) : with(std::integral_constant<int, BR_LOW>{});
-    });
+    auto with = [&](auto rows) { return rb.dscale ? run(rows, std::true_type{}) : run(rows, std::false_type{}); };
+    return ba == BG ? with(std::integral_constant<int, BG>{}) : with(std::integral_constant<int, BR_LOW>{});
 }
 
 // First launch of the backward pass: t (row-major, for the t . N kernel of the tile engine) and dC.  `dc`: where the

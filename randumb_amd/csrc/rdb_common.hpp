@@ -4,7 +4,6 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-#include <type_traits>
 
 #include "../../include/randumb_hip.h"
 
@@ -156,23 +155,6 @@ template <class V> __device__ __forceinline__ void store_stream(V *dst, const V 
 // loaded with device scope (SCOPE_DEVICE below: write-through, and read from memory), as the tags are.
 constexpr int SYNC_SPIN_LIMIT = 1 << 17;
 constexpr int SCOPE_DEVICE = 16;   // cache-policy argument of the raw buffer loads and stores: sc1
-constexpr int STORE_STREAM = 2;    // nt
-
-// f(cache policy, as std::integral_constant) of the stores of a result [tokens x features], leading dimension ld, that this library does not read
-// again.  Rows of whole lines of 128 bytes: written through while the layer's activations (pass_bytes: one side's and the other's) are a
-// quarter of the 256 MB of the memory-side cache, which then takes the lines and hands them to the next reader, and non-temporal above that,
-// where lines that linger displace what the pass reads.  Neither waits dirty in L2 for a write-back at the kernel's end, as plain stores do
-// (8192 tokens x 768 -> 3072, forward: plain 29.4 us, non-temporal 27.0).  us of a training step, non-temporal and through: 8192 x 768 -> 3072, k = 256
-// (60 MB): 71.2, 70.3; 4096 x 1024 -> 8192, k = 128 (72): 71.5, 70.1; 8192 x 1024 -> 4096 (80): 76.2, 74.2; 5000 x 2048 -> 5000 (67): 72.5, 73.7; 8192 x
-// 1024 -> 5120 (96): 82.2, 88.2; 8192 x 1024 -> 8192 (144): 115.6, 130.0; forward alone, 800 x 2048 -> 8192: 24.7, 23.6; 2048 x 4096 -> 11008: 36.9, 35.0;
-// GPT-2 small 7960, 7930.  Other rows leave with plain stores: a pair of neighbouring 128-byte pieces shares a line there, and a
-// streamed part of a line is a read and a write of memory (7186 tokens x 264 -> 5384: forward 63.5 -> 30.6 us; 4096 x 264 -> 5400: 33.6 -> 18;
-// -> 5408, halves of lines: 18.4 -> 17.4; -> 5440, whole lines: 17.0 streamed, 17.2 plain; dx of 4096 x 3208 -> 520: 16.4 -> 8.9).
-template <class F> inline int with_store_policy(const void *result, int64_t ld, int64_t pass_bytes, F &&f)
-{
-    if (ld % 64 != 0 || ((uintptr_t)result & 127) != 0) return f(std::integral_constant<int, 0>{});
-    return pass_bytes <= (64ll << 20) ? f(std::integral_constant<int, SCOPE_DEVICE>{}) : f(std::integral_constant<int, STORE_STREAM>{});
-}
 
 // What a waiting block needs besides its slots: how long to wait and where to report that it gave up.
 struct SyncWait {

@@ -405,7 +405,7 @@ static int64_t tns_table_bytes(const rdb_linear_desc *d, int num_cus)
     const int64_t bytes = cdiv(d->in_f, 32) * 32 * cdiv(d->k, 64) * 64 * (int64_t)sizeof(bf16_t);
     if (d->k <= 128 || d->k > ST_KMAX || bytes >= (1ll << 30)) return 0;
     StParams q;
-    make_stationary_grid(q, d->tokens, d->in_f, d->out_f, num_cus);
+    make_stationary_grid(q, d->tokens, d->in_f, num_cus);
     return q.tiles_t >= 12 && q.units_per_split >= (d->out_f <= 2 * d->in_f ? 2 : 3) ? bytes : 0;
 }
 // Scratch of the regrouped backward pass that it can do without: the ranges' sums and behind them, or later in their place (k > 256), N^T for dx = t . N
@@ -433,7 +433,7 @@ static int make_tns_params(StParams &q, void *dx, int64_t lddx, const void *t, c
     q.ldy = lddx;
     q.k = (int)d->k;
     q.seed = d->seed;
-    return make_stationary_grid(q, d->tokens, d->in_f, d->out_f, num_cus);
+    return make_stationary_grid(q, d->tokens, d->in_f, num_cus);
 }
 
 // Returns RDB_E_UNSUPPORTED (without setting an error) when the request does not fit this algorithm.

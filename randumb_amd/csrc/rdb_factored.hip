@@ -649,7 +649,7 @@ static int fill_ys_params(StParams &q, void *y, int64_t ldy, const void *state, 
     q.ldy = ldy;
     q.k = (int)d->k;
     q.seed = 0;
-    return make_stationary_grid(q, d->tokens, d->out_f, d->in_f, num_cus);
+    return make_stationary_grid(q, d->tokens, d->out_f, num_cus);
 }
 
 template <bool BIAS> static int launch_zy(const ZYParams &p, int y_items, hipStream_t s)

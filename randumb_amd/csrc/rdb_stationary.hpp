@@ -16,6 +16,13 @@
 
 namespace rdb {
 
+// Cache policy of the output row stores where rows are whole lines of 128 bytes: non-temporal (y and dx are not read again by this library,
+// and lines that do not linger in L2 need no write-back when the kernel ends: the next launch starts sooner; 8192 tokens x 768 -> 3072,
+// forward 27.0 us, with plain stores 29.4).  Other rows leave with plain stores: a pair of neighbouring 128-byte pieces shares a line there, and a
+// streamed part of a line is a read and a write of memory (7186 tokens x 264 -> 5384: forward 63.5 -> 30.6 us; 4096 x 264 -> 5400: 33.6 -> 18;
+// -> 5408, halves of lines: 18.4 -> 17.4; -> 5440, whole lines: 17.0 streamed, 17.2 plain; dx of 4096 x 3208 -> 520: 16.4 -> 8.9).
+constexpr int Y_STREAM = 2;
+
 constexpr int ST_BT = 256, ST_BO = 64, ST_STG_LD = ST_BO + 8, ST_WAVES = 8, ST_THREADS = ST_WAVES * 64, ST_TW = ST_BT / ST_WAVES;
 constexpr int ST_KMAX = 256;
 
@@ -29,7 +36,6 @@ struct StParams {
     int tokens, out_f, k;
     int tiles_t, splits, units_per_split;
     uint32_t seed;       // noise flavour
-    int64_t pass_bytes;  // of the layer's activations, one side's and the other's (with_store_policy)
     // ZFRAG only: NULL, or slots [token tile of 256][sync_n + 1] that earlier blocks of the same launch set to sync_tag when the
     // tile's share of z is in memory (the last slot of a tile counts the blocks that have seen them)
     unsigned long long *sync;
@@ -347,10 +353,8 @@ inline size_t stationary_smem(int kg)
 }
 
 // Grid of the stationary kernels for [tokens x out_f]: about one block per compute unit.  Returns the number of work items.
-// contracted: the features on the layer's other side
-inline int make_stationary_grid(StParams &q, int64_t tokens, int64_t out_f, int64_t contracted, int num_cus)
+inline int make_stationary_grid(StParams &q, int64_t tokens, int64_t out_f, int num_cus)
 {
-    q.pass_bytes = tokens * (out_f + contracted) * 2;
     q.tokens = (int)tokens;
     q.out_f = (int)out_f;
     q.sync = nullptr;   // the left operand comes from an earlier launch unless the caller says otherwise afterwards
@@ -377,7 +381,8 @@ template <class F> inline int with_stationary_variant(const StParams &q, F &&f)
         default: return f(std::integral_constant<int, 4>{}, aux);
         }
     };
-    return with_store_policy(q.y, q.ldy, q.pass_bytes, with_kg);
+    const bool whole_lines = q.ldy % 64 == 0 && ((uintptr_t)q.y & 127) == 0;
+    return whole_lines ? with_kg(std::integral_constant<int, Y_STREAM>{}) : with_kg(std::integral_constant<int, 0>{});
 }
 
 template <class K> inline int launch_stationary(K kernel, const StParams &q, int items, size_t smem, hipStream_t s, const char *name)

@@ -704,12 +704,13 @@ template <int BA, bool DOT, bool STREAM> __global__ __launch_bounds__(256, 1) vo
         PT pt;
         frag_rows(pt, p.t, p.tokens, p.k, tok0);
         BigRegs<PR, PT> regs2;
-        // x as the accumulators lie: four features of a token a lane (in_f is a multiple of 8: all inside or all outside, which reads as zeros)
+        // x as the accumulators lie: four features of a token a lane (in_f is a multiple of 8: all inside or all outside, which reads as zeros).  A token
+        // behind the last has no offset of its own: with rows far apart the 32-bit product would come round and lie between rows of x.
         uint2 xv[NI][MI][4];
         auto load_x = [&](int ni) __attribute__((always_inline)) {
             const int t = opaque_tid(), wave = t >> 6, lane = t & 63;
             const int tok = tok0 + (wave & 1) * NI * 32 + ni * 32 + (lane & 31), f = a0 + (wave >> 1) * MI * 32 + 4 * (lane >> 5);
-            const uint32_t at = ((uint32_t)tok * (uint32_t)p.ldx + (uint32_t)f) * 2u;   // a token behind the last is behind the buffer's end too
+            const uint32_t at = tok < p.tokens ? ((uint32_t)tok * (uint32_t)p.ldx + (uint32_t)f) * 2u : BUFFER_OOB;
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi)
 #pragma unroll

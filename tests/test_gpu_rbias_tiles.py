@@ -99,3 +99,28 @@ def test_backward_in_one_call_against_float64(T, in_f, out_f, k):
     want = dyd @ C.double() @ N.t() + s.double() * dyd @ R
     assert float((dx.double() - want).norm() / want.norm()) < 6e-3   # N, t, R and dx rounded to bf16 once each, 1.13e-3 as a norm; 2^-9 at most
     assert abs(float(ds[0]) - float((dot * xd).sum())) < 1e-5 * float(dot.norm() * xd.norm())   # fp32 sums
+
+
+# rows of x so far apart that the offset of a token behind the last one, taken in 32 bits, lies between two rows: what is there is no part of the sum
+def test_scale_gradient_reads_no_gap_between_rows():
+    from randumb_amd import _lib, hip
+
+    T, in_f, out_f, k, ldx = 16, 32768, 16, 24, 2**25 - 8
+    print(f"case rbias backward, rows of x {ldx} apart", flush=True)
+    assert T * ldx < 2**29 and 65 * ldx * 2 - 2**32 < ldx * 2   # taken as it is; the 66th row of a tile of 128
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device="cuda").manual_seed(T)
+    ref = ctypes.byref(hip._proj_desc(T, in_f, out_f, k, 9))
+    n = lib.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_BWD_PROJECTED_RBIAS, ref)
+    assert n > 0
+    far = torch.full(((T - 1) * ldx + in_f,), float("nan"), device="cuda", dtype=torch.bfloat16)
+    x = far.as_strided((T, in_f), (ldx, 1))
+    x.copy_(torch.randn(T, in_f, device="cuda", generator=g))
+    C, dy = (torch.randn(out_f, k, device="cuda", generator=g) * k**-0.5).bfloat16(), torch.randn(T, out_f, device="cuda", generator=g).bfloat16()
+    s, ws, ds = torch.tensor([0.37], device="cuda").bfloat16(), torch.empty(n, dtype=torch.uint8, device="cuda"), torch.empty(1, device="cuda")
+    state = hip.linear_project(x.contiguous(), k, out_f, 9, C)
+    dx, dc = torch.empty(T, in_f, device="cuda", dtype=torch.bfloat16), torch.empty_like(C)
+    assert lib.rdb_linear_bwd_projected_rbias(dx.data_ptr(), in_f, dc.data_ptr(), _lib.RDB_BF16, ds.data_ptr(), _lib.RDB_F32, dy.data_ptr(), out_f, state.data_ptr(),
+                                              x.data_ptr(), ldx, C.data_ptr(), s.data_ptr(), ref, ws.data_ptr(), n, stream) == 0
+    dot = dy.double() @ hip.sq5_fill_1d(out_f * in_f, 9).view(out_f, in_f).bfloat16().double()
+    assert abs(float(ds) - float((dot * x.double()).sum())) < 1e-5 * float(dot.norm() * x.double().norm())   # fp32 sums

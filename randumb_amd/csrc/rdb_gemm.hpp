@@ -165,9 +165,16 @@ template <int ROWS, int BK, int LAYOUT> struct GlobalOperand {
         kk = Tile::thread_kk();
         q = Tile::pieces(ld, row0, nrows, kb);
         // M_CONT: contraction indices are rows of the source, so clipping the buffer at row klim makes the hardware bounds
-        // check zero everything from klim on.  K_CONT clips per thread in load_piece().
+        // check zero everything from klim on.  K_CONT clips per thread in load_piece().  Rows of the first stage that lie past klim are
+        // marked as well: with few rows far apart their 32-bit offset would come round into the buffer (15 rows or fewer, over 2^25 elements
+        // apart).  In a later stage row klim + BK is at most twice as far as the last one, below 2^31 bytes.
         int64_t bytes = extent * 2;
         if (LAYOUT == M_CONT && (int64_t)klim * ld * 2 < bytes) bytes = (int64_t)klim * ld * 2;
+        if (LAYOUT == M_CONT) {
+#pragma unroll
+            for (int p = 0; p < Tile::PER_THREAD; ++p)
+                if (kb + (p * 256 + (int)threadIdx.x) / (ROWS / 8) >= klim) q.off[p] = BUFFER_OOB;
+        }
         rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(src), 0, (int)bytes, 0x00020000);
     }
     __device__ __forceinline__ void load_piece(f32x4 &reg, int p, int stage) const

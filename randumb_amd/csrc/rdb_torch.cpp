@@ -141,6 +141,10 @@ Tensor near_act(const Tensor &t0)
     return t.size(0) * t.stride(0) >= (1ll << 29) ? t.contiguous() : t;
 }
 
+// ... of the input as a backward pass gets it back, in the gradient's dtype, as the kernels that read both by address take it (hooks on saved tensors may
+// keep it in another one)
+Tensor near_input(const Tensor &x, const Tensor &dy) { return near_act(x.to(dy.scalar_type())); }
+
 Tensor bytes(int64_t n, const Tensor &like) { return n > 0 ? at::empty({n}, like.options().dtype(at::kByte)) : Tensor(); }
 void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
 
@@ -426,7 +430,7 @@ class OneCallLinear : public Function<OneCallLinear> {
         if (kept.defined()) {
             if (want_dx || want_dc || want_sb) {
                 const c10::OptionalDeviceGuard guard(dy.device());
-                const Tensor c = coefs.contiguous(), xs = want_sb ? near_act(x) : Tensor(), s = has_sb ? sb.to(c.scalar_type()) : Tensor();
+                const Tensor c = coefs.contiguous(), xs = want_sb ? near_input(x, dy) : Tensor(), s = has_sb ? sb.to(c.scalar_type()) : Tensor();
                 const rdb_linear_desc d = desc(dy, l, c);
                 const int64_t kept_bytes = rdb_linear_kept_bytes(&d);   // 0: the coefficients came back in another dtype
                 restored_values(who, kept, dy, at::kByte, kept_bytes ? kept_bytes : -1);
@@ -541,7 +545,7 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         // with the fused random bias: both shares of dx, all gradients, in one call where the layer has such a form (it refuses what the two calls refuse)
         const int64_t both_shares = has_sb && !f32 && want_dx && want_dc ? rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_PROJECTED_RBIAS, &d) : 0;
         if (both_shares) {
-            const Tensor x = want_sb ? near_act(saved[3]) : Tensor(), sb = native(scale_bias).to(at::kBFloat16), ws = bytes(both_shares, dy);
+            const Tensor x = want_sb ? near_input(saved[3], dy) : Tensor(), sb = native(scale_bias).to(at::kBFloat16), ws = bytes(both_shares, dy);
             const auto dt = scale_bias.scalar_type() == at::kBFloat16 ? at::kBFloat16 : at::kFloat;
             dx = at::empty({dy.size(0), l.in_f}, dy.options());
             dc = at::empty({c.size(0), c.size(1)}, dy.options().dtype(at::kBFloat16));
@@ -571,7 +575,7 @@ class ProjectedLinear : public Function<ProjectedLinear> {
             dc = dc.to(c.scalar_type());
         }
         if (has_sb && dx.defined() && !both_shares) {
-            const Tensor x = near_act(saved[3]), sb = native(scale_bias).to(at::kBFloat16);
+            const Tensor x = near_input(saved[3], dy), sb = native(scale_bias).to(at::kBFloat16);
             const rdb_linear_desc r = rbias_desc(dy, l);
             const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_RBIAS_BWD_FULL, &r);
             const Tensor ws = bytes(need, dy);

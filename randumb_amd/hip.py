@@ -477,7 +477,7 @@ def linear_rbias_bwd_(dx: torch.Tensor, dy: torch.Tensor, x: Optional[torch.Tens
             _lib.check(L.rdb_linear_rbias_bwd(_p(dx), dx.stride(0), None, _p(dy), dy.stride(0), None, 0, _p(sb), ctypes.byref(d), None, 0,
                                               _stream(dy.device)), "rdb_linear_rbias_bwd")
             return None
-        x = _act(x)
+        x = _act(x.to(dy.dtype))
         ws_bytes = int(L.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_RBIAS_BWD, ctypes.byref(d)))
         ws = _workspace(ws_bytes, dy.device)
         ds = torch.empty((1,), dtype=torch.float32, device=dy.device)

@@ -894,7 +894,7 @@ NoiseTable rbias_dx_table(const RBiasDx &rb, const rdb_linear_desc *d)
 {
     return noise_frag_table(rb.r, d->in_f, d->out_f, SQ5_N1, (uint32_t)d->in_f * SQ5_N1, d->seed, rb.arrived);
 }
-NoiseTable noise_dx_table(const RBiasDx &rb, const rdb_linear_desc *d) { return noise_frag_table(rb.n, d->in_f, d->k, PN1, SQ5_N1, d->seed, nullptr, 1.0f); }
+NoiseTable noise_dx_table(bf16_t *n, const rdb_linear_desc *d) { return noise_frag_table(n, d->in_f, d->k, PN1, SQ5_N1, d->seed, nullptr, 1.0f); }
 
 // Scratch for N^T where dx = t . N takes it from memory; 0: where it does not.
 int64_t dx_big_table_bytes(const rdb_linear_desc *d, int num_cus)

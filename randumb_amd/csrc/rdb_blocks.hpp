@@ -134,7 +134,7 @@ struct RBiasDx {
     int dscale_dtype;
     float *dots;           // one share a tile
     unsigned int *arrived; // a word
-    bf16_t *r, *n;         // room for R and N^T in fragment order (without a random bias: n alone)
+    bf16_t *r, *n;         // room for R and N^T in fragment order
 };
 
 __device__ __forceinline__ void red_block(const RedParams &p, int block, int nblocks)
@@ -241,7 +241,7 @@ int linear_z_big(void *state, const void *x, int64_t ldx, const void *coef, void
                  hipStream_t s);
 int64_t dx_big_table_bytes(const rdb_linear_desc *d, int num_cus);
 NoiseTable rbias_dx_table(const RBiasDx &rb, const rdb_linear_desc *d);
-NoiseTable noise_dx_table(const RBiasDx &rb, const rdb_linear_desc *d);
+NoiseTable noise_dx_table(bf16_t *n, const rdb_linear_desc *d);
 int linear_dx_rbias_big(void *dx, int64_t lddx, const void *t, const void *dy, int64_t lddy, const RBiasDx &rb, const RedParams *red, const rdb_linear_desc *d,
                         int num_cus, hipStream_t s);
 int linear_tn_big(void *dx, int64_t lddx, const void *t, void *table, const rdb_linear_desc *d, int num_cus, hipStream_t s);

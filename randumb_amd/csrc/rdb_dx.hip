@@ -409,13 +409,14 @@ static int64_t tns_table_bytes(const rdb_linear_desc *d, int num_cus)
     return q.tiles_t >= 12 && q.units_per_split >= (d->out_f <= 2 * d->in_f ? 2 : 3) ? bytes : 0;
 }
 // Scratch of the regrouped backward pass that it can do without: the ranges' sums and behind them, or later in their place (k > 256), N^T for dx = t . N
-int64_t linear_bwd_projected_extra(const rdb_linear_desc *d, int num_cus)
+// (table false: for the random bias's form, which has room for N^T of its own)
+int64_t linear_bwd_projected_extra(const rdb_linear_desc *d, int num_cus, bool table)
 {
     if (!dx_factored_ok(d)) return 0;
     int len;
     const int ranges = dyc_ranges(d, num_cus, &len);
     const int64_t part = ranges > 1 ? align256(ranges * d->tokens * d->k * (int64_t)sizeof(float)) : 0;
-    return std::max<int64_t>(part + tns_table_bytes(d, num_cus), dx_big_table_bytes(d, num_cus));
+    return table ? std::max<int64_t>(part + tns_table_bytes(d, num_cus), dx_big_table_bytes(d, num_cus)) : part;
 }
 
 // t . N with t in registers applies when k is short enough and dx fits a buffer descriptor.
@@ -519,9 +520,9 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
         if (a.dyc.ranges > 1 && workspace_bytes >= base + align256(a.dyc.ranges * d->tokens * d->k * (int64_t)sizeof(float)))
             a.dyc.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + base);
         const int64_t table_at = base + (a.dyc.part ? align256(a.dyc.ranges * d->tokens * d->k * (int64_t)sizeof(float)) : 0), table_n = tns_table_bytes(d, num_cus);
-        RBiasDx nt = {};
+        bf16_t *n = rb ? rb->n : nullptr;   // N^T in memory, or none
         if (!rb && table_n && tn_stationary_ok(d, lddx) && workspace_bytes >= table_at + table_n)
-            nt.n = reinterpret_cast<bf16_t *>(static_cast<char *>(workspace) + table_at);
+            n = reinterpret_cast<bf16_t *>(static_cast<char *>(workspace) + table_at);
         a.dc_blocks = xcd_grid_size(dc_items);
         int rc = RDB_OK;
         const int red_splits = big ? 1 : a.dc.splits;
@@ -534,8 +535,8 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             size_t smem = smem_dc > smem_dyc ? smem_dc : smem_dyc;
             const int dyc_items = p1.tiles_c * p1.tiles_t * (a.dyc.part ? a.dyc.ranges : 1);
             const int blocks = a.dc_blocks + xcd_grid_size(dyc_items);
-            if (rb || nt.n) {
-                const BwdTables tables = {rb ? rbias_dx_table(*rb, d) : NoiseTable{}, noise_dx_table(rb ? *rb : nt, d), blocks};
+            if (n) {
+                const BwdTables tables = {rb ? rbias_dx_table(*rb, d) : NoiseTable{}, noise_dx_table(n, d), blocks};
                 auto kernel = dyc_items * 2 <= num_cus ? bwd_dc_dyc_kernel<2, true> : bwd_dc_dyc_kernel<1, true>;
                 if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem, "bwd_dc_dyc_kernel")) return rl;
                 kernel<<<blocks + table_blocks(tables.r.pieces + tables.n.pieces, num_cus), 256, smem, s>>>(a, tables);
@@ -580,10 +581,10 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             if (spare > 0 && rblocks > spare && std::min(rblocks, num_cus / 2) <= 2 * spare) rblocks = spare;
             if (rblocks < 1) rblocks = 1;
             if (direct) rblocks = 0;
-            bs.tn.coef = nt.n;
+            bs.tn.coef = n;
             return with_stationary_variant(bs.tn, [&](auto kg, auto aux) {
                 constexpr int KG = decltype(kg)::value, AUX = decltype(aux)::value;
-                auto kernel = nt.n ? bwd_tns_red_kernel<KG, AUX, (KG > 2)> : bwd_tns_red_kernel<KG, AUX, false>;   // no table up to k = 128
+                auto kernel = n ? bwd_tns_red_kernel<KG, AUX, (KG > 2)> : bwd_tns_red_kernel<KG, AUX, false>;   // no table up to k = 128
                 const size_t smem_s = stationary_smem(kg);
                 if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem_s, "bwd_tns_red_kernel")) return rl;
                 kernel<<<bs.tn_blocks + rblocks, ST_THREADS, smem_s, s>>>(bs);

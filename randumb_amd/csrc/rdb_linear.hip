@@ -354,7 +354,7 @@ int big_tiles_mode();
 bool big_bwd_applies(const rdb_linear_desc *d, int num_cus);
 int linear_bwd_big(void *t, void *dc, bool dc_bf16, const void *dy, int64_t lddy, const void *state, const void *coef, const rdb_linear_desc *d,
                    int num_cus, bool want_t, bool want_dc, hipStream_t s);
-int64_t linear_bwd_projected_extra(const rdb_linear_desc *d, int num_cus);
+int64_t linear_bwd_projected_extra(const rdb_linear_desc *d, int num_cus, bool table = true);
 
 // rdb_rbias.hip
 int linear_dx_rbias_add(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *scale_bias, const rdb_linear_desc *d, hipStream_t s, void *table = nullptr, int64_t table_bytes = 0);
@@ -1313,19 +1313,20 @@ static int bwd_projected_entry(const char *who, void *dx, int64_t lddx, void *dc
     return RDB_OK;
 }
 
-// Workspace of the backward pass of a layer with a fused random bias as two launches: that of the low-rank share, then the tiles' shares of the
-// scale's gradient, a word to count in, R and N^T.  bytes 0: no such form (too few tiles, or a contraction that does not stay in registers).
+// Workspace of the backward pass of a layer with a fused random bias as two launches: that of the low-rank share without its N^T, then the tiles' shares
+// of the scale's gradient, a word to count in, R and N^T.  bytes 0: no such form (too few tiles, or a contraction that does not stay in registers).
 static BwdRBiasRoom bwd_projected_rbias_room(const rdb_linear_desc *d)
 {
     BwdRBiasRoom r = {};
     const int cus = num_compute_units();
     if (d->act_dtype != RDB_BF16 || d->coef_dtype != RDB_BF16 || d->coef_rows == 0 || d->sO != d->in_f || d->sI != 1 || d->k > 256 || chunk_plan(d).nchunks != 1) return r;
-    const int64_t table = rbias_big_table_bytes(d, d->in_f, cus), base = rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_PROJECTED_TO, d);
+    if (d->algo == RDB_ALGO_TILE || d->algo == RDB_ALGO_STRIP) return r;
+    const int64_t table = rbias_big_table_bytes(d, d->in_f, cus), base = bwd_projected_workspace(d, true);
     if (table <= 0 || base <= 0 || d->tokens * d->in_f >= (1ll << 29) || d->tokens * d->out_f >= (1ll << 29) ||
         rbias_big_tiles(d->in_f, d->tokens, cus) > linear_dx_rbias_dot_floats(d))
         return r;
     auto up = [](int64_t n) { return (n + 255) / 256 * 256; };
-    r.dots = up(base);
+    r.dots = up(base) + up(linear_bwd_projected_extra(d, cus, false));
     r.arrived = r.dots + rbias_dot_room(d);
     r.r = r.arrived + 256;
     r.n = r.r + up(table);

@@ -58,3 +58,13 @@ def test_short_inputs_of_narrow_layers_take_one_range():
     for in_f, ranges in ((1040, False), (1344, False), (1352, True)):   # 17, 21 and 22 stages of 64 features
         n = lib.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_PROJECT, ctypes.byref(_desc(2304, in_f, 32, 16, _lib.RDB_BF16)))
         assert (n > 0) == ranges, (in_f, n)
+
+
+@pytest.mark.parametrize("T,in_f,out_f,k", [(8192, 3072, 768, 256), (8192, 768, 768, 200), (6000, 2048, 6144, 200), (6000, 1000, 1000, 192), (4096, 8192, 1024, 136)])
+def test_the_backward_pass_with_a_random_bias_has_room_for_the_noise_once(T, in_f, out_f, k):
+    """Its scratch: that of the layer without the bias, which holds N^T for these, and R, the shares of the scale's gradient and a word to count in."""
+    lib, RBIAS_BWD_FULL = _lib.load(), 10
+    d, rbias = _desc(T, in_f, out_f, k, _lib.RDB_BF16), _desc(T, in_f, out_f, 8, _lib.RDB_BF16)
+    ops = (_lib.RDB_OP_LINEAR_BWD_PROJECTED_RBIAS, _lib.RDB_OP_LINEAR_BWD_PROJECTED_TO, RBIAS_BWD_FULL)
+    both, base, more = (lib.rdb_linear_workspace_bytes(op, ctypes.byref(x)) for op, x in zip(ops, (d, d, rbias)))
+    assert both and more > 2 * in_f * out_f and both <= base + more + 3 * 256, (both, base, more)

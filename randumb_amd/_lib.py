@@ -18,6 +18,9 @@ RDB_OP_LINEAR_FWD, RDB_OP_LINEAR_BWD_DX, RDB_OP_LINEAR_BWD_DCOEF, RDB_OP_LINEAR_
 RDB_OP_LINEAR_BWD_DX_DSCALE = 5
 RDB_OP_LINEAR_RBIAS_BWD = 6
 RDB_OP_LINEAR_BWD_KEPT = 7
+RDB_OP_LINEAR_RBIAS_FWD = 8
+RDB_OP_LINEAR_PROJECT_FWD_RBIAS = 9
+RDB_OP_LINEAR_RBIAS_BWD_FULL = 10
 RDB_OP_LINEAR_PROJECT = 11
 RDB_OP_LINEAR_FWD_KEPT = 12
 RDB_OP_LINEAR_BWD_PROJECTED_RBIAS = 13

@@ -445,9 +445,10 @@ def linear_rbias_supported(in_f: int, out_f: int, dtype) -> bool:
     return dtype == torch.bfloat16 and in_f % 8 == 0 and out_f % 8 == 0
 
 
-def linear_rbias_fwd_(y: torch.Tensor, x: torch.Tensor, scale_bias: torch.Tensor, in_f: int, out_f: int, seed: int) -> torch.Tensor:
+def linear_rbias_fwd_(y: torch.Tensor, x: torch.Tensor, scale_bias: torch.Tensor, in_f: int, out_f: int, seed: int, scratch: bool = False) -> torch.Tensor:
     """In place: ``y += scale_bias * x @ R.T`` with ``R[o, i] = noise1d(o * in_f + i)``, the fused random bias of a weight
-    ``W = C.N + s.R`` (src/rten_cpp/RandumbTensor.py:286-289), on top of a ``y`` that holds the low-rank share.  bf16."""
+    ``W = C.N + s.R`` (src/rten_cpp/RandumbTensor.py:286-289), on top of a ``y`` that holds the low-rank share.  bf16.  ``scratch``: with
+    room for R in memory or for the sums of ranges of the contraction, as the extension module calls it."""
     _need_gpu("linear_rbias_fwd_", y, x, scale_bias)
     x = _act(x)
     _need_shape("linear_rbias_fwd_", "the input", x, None, in_f)
@@ -455,15 +456,18 @@ def linear_rbias_fwd_(y: torch.Tensor, x: torch.Tensor, scale_bias: torch.Tensor
     sb = _native(scale_bias).to(torch.bfloat16)
     d = _rbias_desc(x.shape[0], in_f, out_f, seed)
     with _on(x.device):
-        _lib.check(_lib.load().rdb_linear_rbias_fwd(_p(y), y.stride(0), _p(x), x.stride(0), _p(sb), ctypes.byref(d), _stream(x.device)),
+        L = _lib.load()
+        ws_bytes = int(L.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_RBIAS_FWD, ctypes.byref(d))) if scratch else 0
+        ws = _workspace(ws_bytes, x.device)
+        _lib.check(L.rdb_linear_rbias_fwd_ws(_p(y), y.stride(0), _p(x), x.stride(0), _p(sb), ctypes.byref(d), _p(ws), ws_bytes, _stream(x.device)),
                    "rdb_linear_rbias_fwd")
     return y
 
 
 def linear_rbias_bwd_(dx: torch.Tensor, dy: torch.Tensor, x: Optional[torch.Tensor], scale_bias: torch.Tensor, in_f: int, out_f: int,
-                      seed: int, want_scale_bias_grad: bool = False) -> Optional[torch.Tensor]:
+                      seed: int, want_scale_bias_grad: bool = False, scratch: bool = False) -> Optional[torch.Tensor]:
     """In place: ``dx += scale_bias * dy @ R``; returns the gradient of the scale, ``<dy @ R, x>`` (fp32, ``(1,)``), from the same
-    pass when asked for (``x`` is needed then only)."""
+    pass when asked for (``x`` is needed then only).  ``scratch`` as in :func:`linear_rbias_fwd_`."""
     _need_gpu("linear_rbias_bwd_", dx, dy, scale_bias, x if want_scale_bias_grad else None)
     dy = _act(dy)
     _need_shape("linear_rbias_bwd_", "the gradient", dy, None, out_f)
@@ -473,13 +477,14 @@ def linear_rbias_bwd_(dx: torch.Tensor, dy: torch.Tensor, x: Optional[torch.Tens
     d = _rbias_desc(dy.shape[0], in_f, out_f, seed)
     L = _lib.load()
     with _on(dy.device):
+        op = _lib.RDB_OP_LINEAR_RBIAS_BWD_FULL if scratch else _lib.RDB_OP_LINEAR_RBIAS_BWD
+        ws_bytes = int(L.rdb_linear_workspace_bytes(op, ctypes.byref(d))) if scratch or want_scale_bias_grad else 0
+        ws = _workspace(ws_bytes, dy.device)
         if not want_scale_bias_grad:
-            _lib.check(L.rdb_linear_rbias_bwd(_p(dx), dx.stride(0), None, _p(dy), dy.stride(0), None, 0, _p(sb), ctypes.byref(d), None, 0,
+            _lib.check(L.rdb_linear_rbias_bwd(_p(dx), dx.stride(0), None, _p(dy), dy.stride(0), None, 0, _p(sb), ctypes.byref(d), _p(ws), ws_bytes,
                                               _stream(dy.device)), "rdb_linear_rbias_bwd")
             return None
         x = _act(x.to(dy.dtype))
-        ws_bytes = int(L.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_RBIAS_BWD, ctypes.byref(d)))
-        ws = _workspace(ws_bytes, dy.device)
         ds = torch.empty((1,), dtype=torch.float32, device=dy.device)
         _lib.check(L.rdb_linear_rbias_bwd(_p(dx), dx.stride(0), _p(ds), _p(dy), dy.stride(0), _p(x), x.stride(0), _p(sb), ctypes.byref(d),
                                           _p(ws), ws_bytes, _stream(dy.device)), "rdb_linear_rbias_bwd")
@@ -625,14 +630,17 @@ def linear_project(x: torch.Tensor, k: int, out_f: int, seed: int, coef: Optiona
     return state
 
 
-def linear_project_fwd(x: torch.Tensor, coef: torch.Tensor, seed: int, bias: Optional[torch.Tensor] = None):
+def linear_project_fwd(x: torch.Tensor, coef: torch.Tensor, seed: int, bias: Optional[torch.Tensor] = None, scale_bias: Optional[torch.Tensor] = None):
     """``(y, state)``: :func:`linear_project` (with ``coef``) and :func:`linear_fwd_projected` in one call, for k <= 256 in a
-    single kernel launch; the forward pass of a training step, ``state`` being what it saves for backward."""
-    _need_gpu("linear_project_fwd", x, coef, bias)
+    single kernel launch; the forward pass of a training step, ``state`` being what it saves for backward.  ``scale_bias``: with the fused
+    random bias's share (bf16), in one product where the library has such a form, by :func:`linear_rbias_fwd_` otherwise."""
+    _need_gpu("linear_project_fwd", x, coef, bias, scale_bias)
     x = _act(x)
     c = coef if coef.is_contiguous() else coef.contiguous()
     if x.dtype != c.dtype or x.dtype not in _DT:
         raise ValueError("linear_project_fwd computes in bf16 or in fp32: activations and coefficients in one of them")
+    if scale_bias is not None and x.dtype != torch.bfloat16:
+        raise ValueError("linear_project_fwd: the fused random bias has this form in bf16 only")
     out_f, k = c.shape
     tokens = x.shape[0]
     _need_bias("linear_project_fwd", bias, out_f)
@@ -646,12 +654,20 @@ def linear_project_fwd(x: torch.Tensor, coef: torch.Tensor, seed: int, bias: Opt
     y = torch.empty((tokens, out_f), dtype=x.dtype, device=dev)
     with _on(dev):
         st = _stream(dev)
-        ws = _workspace(pl.project_bytes, dev)
-        rc = L.rdb_linear_project_fwd_ws(y.data_ptr(), out_f, state.data_ptr(), x.data_ptr(), x.stride(0), c.data_ptr(),
-                                         None if b is None else b.data_ptr(), pl.ref, _p(ws), pl.project_bytes, st)
+        one_product = 0 if scale_bias is None else int(L.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_PROJECT_FWD_RBIAS, pl.ref))
+        ws = _workspace(one_product or pl.project_bytes, dev)
+        if one_product:
+            sb = _native(scale_bias).to(torch.bfloat16)
+            rc = L.rdb_linear_project_fwd_rbias(y.data_ptr(), out_f, state.data_ptr(), x.data_ptr(), x.stride(0), c.data_ptr(), sb.data_ptr(),
+                                                None if b is None else b.data_ptr(), pl.ref, _p(ws), one_product, st)
+        else:
+            rc = L.rdb_linear_project_fwd_ws(y.data_ptr(), out_f, state.data_ptr(), x.data_ptr(), x.stride(0), c.data_ptr(),
+                                             None if b is None else b.data_ptr(), pl.ref, _p(ws), pl.project_bytes, st)
         if rc:
             _lib.check(rc, "rdb_linear_project_fwd")
         _watch(dev).tick(st)
+    if scale_bias is not None and not one_product:
+        linear_rbias_fwd_(y, x, scale_bias, x.shape[1], out_f, seed, scratch=True)
     return y, state
 
 
@@ -802,6 +818,38 @@ def linear_bwd_projected(dy: torch.Tensor, state: torch.Tensor, coef: torch.Tens
     if rc:
         _lib.check(rc, "rdb_linear_bwd_projected")
     return dx, (dcoef if dcoef.dtype == dcoef_dtype else dcoef.to(dcoef_dtype))
+
+
+def linear_bwd_projected_rbias(dy: torch.Tensor, state: torch.Tensor, x: Optional[torch.Tensor], coef: torch.Tensor, scale_bias: torch.Tensor, in_f: int, seed: int,
+                               want_scale_bias_grad: bool = False):
+    """``(dx, dcoef, ds)`` of a bf16 layer with the fused random bias from the projection state, both shares of ``dx`` in one product and
+    rounded once, the gradients in bf16 (``ds``, with ``want_scale_bias_grad`` alone, for which ``x`` is needed, in fp32).  ``None`` where the
+    library has no such form: :func:`linear_bwd_projected` and :func:`linear_rbias_bwd_` then."""
+    _need_gpu("linear_bwd_projected_rbias", dy, state, coef, scale_bias, x if want_scale_bias_grad else None)
+    dy, c = _act(dy), _native(coef)
+    out_f, k = c.shape
+    tokens, dev = dy.shape[0], dy.device
+    _need_shape("linear_bwd_projected_rbias", "the gradient", dy, None, out_f)
+    _need_shape("linear_bwd_projected_rbias", "the input", x if want_scale_bias_grad else None, tokens, in_f)
+    if dy.dtype != torch.bfloat16 or c.dtype != torch.bfloat16:
+        return None
+    pl, L = _plan(tokens, in_f, out_f, k, seed), _lib.load()
+    ws_bytes = int(L.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_BWD_PROJECTED_RBIAS, pl.ref))
+    if ws_bytes <= 0:
+        return None
+    _check_state(state, pl.desc, "linear_bwd_projected_rbias")
+    if CHECK_STATE_COEF:
+        check_state_coef(state, c, in_f)
+    x = _act(x.to(dy.dtype)) if want_scale_bias_grad else None
+    sb = _native(scale_bias).to(torch.bfloat16)
+    dx, dcoef = torch.empty((tokens, in_f), dtype=dy.dtype, device=dev), torch.empty((out_f, k), dtype=c.dtype, device=dev)
+    ds = torch.empty((1,), dtype=torch.float32, device=dev) if want_scale_bias_grad else None
+    with _on(dev):
+        ws = _workspace(ws_bytes, dev)
+        rc = L.rdb_linear_bwd_projected_rbias(_p(dx), in_f, _p(dcoef), RDB_BF16, _p(ds), RDB_F32, _p(dy), dy.stride(0), _p(state), _p(x),
+                                              0 if x is None else x.stride(0), _p(c), _p(sb), pl.ref, _p(ws), ws_bytes, _stream(dev))
+    _lib.check(rc, "rdb_linear_bwd_projected_rbias")
+    return dx, dcoef, ds
 
 
 def set_f32_split(mode: int) -> int:

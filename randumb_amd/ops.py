@@ -342,17 +342,16 @@ class _ProjectedFunction(torch.autograd.Function):
     again (RandumbTensor.py:942-946, 979-990).  Per token the bf16 state holds 4 bytes per coefficient (k rounded up to 64)
     where x holds 2 per input feature, plus once per layer a copy of the coefficients; ``x`` itself usually stays alive too
     (its producer saved it), so ``linear`` takes this function only while the state is at most twice the size of x
-    (``hip.linear_projection_preferred``).  With the fused random bias (``scale_bias``, bf16, eager only) the full-rank share
-    ``s.R`` is added by kernels of its own in both directions and ``x`` is saved as well: the gradient of ``s`` is
-    ``<dy @ R, x>``."""
+    (``hip.linear_projection_preferred``).  With the fused random bias (``scale_bias``, bf16, eager only) ``x`` is saved as well: the
+    gradient of ``s`` is ``<dy @ R, x>``.  The full-rank share ``s.R`` is part of the same product in layers with many tiles and is added by
+    kernels of its own in the others, in both directions: the library says which, and the extension module asks it the same."""
 
     @staticmethod
     def forward(ctx, x, coefs, in_features, out_features, seed, bias, scale_bias=None):
         # eagerly: straight to the library (the operator wrappers of torch.library cost more host time than the layer's
         # kernels take); under torch.compile: through the registered operators, which it can trace
-        y, state = linear_project_fwd(x, coefs, seed, bias) if _tracing() else hip.linear_project_fwd(x, coefs, seed, _dense(bias))
+        y, state = linear_project_fwd(x, coefs, seed, bias) if _tracing() else hip.linear_project_fwd(x, coefs, seed, _dense(bias), scale_bias)
         if scale_bias is not None:
-            hip.linear_rbias_fwd_(y, x, scale_bias, in_features, out_features, seed)
             ctx.save_for_backward(state, coefs, scale_bias, x)
         else:
             ctx.save_for_backward(state, coefs)
@@ -371,8 +370,8 @@ class _ProjectedFunction(torch.autograd.Function):
     @staticmethod
     @torch.no_grad()
     def _gradients(ctx, dy):
-        state, coefs = ctx.saved_tensors[:2]
-        scale_bias, x = ctx.saved_tensors[2:] if len(ctx.saved_tensors) == 4 else (None, None)
+        saved = ctx.saved_tensors
+        state, coefs, scale_bias, x = saved if len(saved) == 4 else (*saved, None, None)
         in_f, out_f, seed = ctx.meta
         if dy.stride(-1) != 1 or dy.stride(0) < dy.shape[1] or dy.stride(0) % 8 or dy.data_ptr() % 16:
             dy = dy.contiguous()   # the kernels read rows with a leading dimension; anything else is copied
@@ -380,7 +379,14 @@ class _ProjectedFunction(torch.autograd.Function):
         direct = not _tracing()
         want_sb = scale_bias is not None and ctx.needs_input_grad[6]
         want_dx = ctx.needs_input_grad[0] or want_sb   # the gradient of the scale comes out of the random-bias share of dx
-        if want_dx and ctx.needs_input_grad[1]:
+        both_shares = None
+        if scale_bias is not None and want_dx and ctx.needs_input_grad[1]:
+            both_shares = hip.linear_bwd_projected_rbias(dy, state, x, coefs, scale_bias, in_f, seed, want_scale_bias_grad=want_sb)
+        if both_shares is not None:
+            dx, dcoefs, ds = both_shares
+            if want_sb:
+                dsb = ds.to(scale_bias.dtype)
+        elif want_dx and ctx.needs_input_grad[1]:
             if direct:   # the sums leave the kernel in the coefficients' dtype: no cast afterwards
                 dx, dcoefs = hip.linear_bwd_projected(dy, state, coefs, in_f, seed, dcoef_dtype=coefs.dtype)
             else:
@@ -396,8 +402,8 @@ class _ProjectedFunction(torch.autograd.Function):
                 dc = (hip.linear_bwd_dcoef_projected(dy, state, coefs.shape[1], in_f, seed) if direct
                       else linear_bwd_dcoef_projected(dy, state, coefs.shape[1], in_f, seed))
                 dcoefs = dc.to(coefs.dtype)
-        if scale_bias is not None and dx is not None:
-            ds = hip.linear_rbias_bwd_(dx, dy, x, scale_bias, in_f, out_f, seed, want_scale_bias_grad=want_sb)
+        if scale_bias is not None and dx is not None and both_shares is None:
+            ds = hip.linear_rbias_bwd_(dx, dy, x, scale_bias, in_f, out_f, seed, want_scale_bias_grad=want_sb, scratch=True)
             if want_sb:
                 dsb = ds.to(scale_bias.dtype)
         return dx if ctx.needs_input_grad[0] else None, dcoefs, dsb

@@ -105,7 +105,8 @@ def test_the_operators_refuse_sizes_that_are_not_the_layers():
                  lambda: hip.linear_bwd_dcoef(dy, _fake(5, IN), K, OUT, IN, OUT, IN, 1, 3), lambda: hip.linear_bwd_dcoef(_fake(4, 8), x, K, OUT, IN, OUT, IN, 1, 3),
                  lambda: hip.linear_project_fwd(x, c, 3, bias=_fake(OUT + 8)), lambda: hip.linear_rbias_fwd_(_fake(3, OUT), x, one, IN, OUT, 3),
                  lambda: hip.linear_rbias_bwd_(_fake(4, IN), dy, _fake(4, OUT), one, IN, OUT, 3, want_scale_bias_grad=True),
-                 lambda: hip.linear_bwd_projected(_fake(4, 8), _fake(4, 8), c, IN, 3)):
+                 lambda: hip.linear_bwd_projected(_fake(4, 8), _fake(4, 8), c, IN, 3), lambda: hip.linear_bwd_projected_rbias(_fake(4, 8), _fake(4, 8), None, c, one, IN, 3),
+                 lambda: hip.linear_bwd_projected_rbias(dy, _fake(4, 8), _fake(4, 8), c, one, IN, 3, want_scale_bias_grad=True)):
         with pytest.raises(RuntimeError, match="must have"):
             call()
 

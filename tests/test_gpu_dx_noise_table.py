@@ -8,8 +8,10 @@ pytestmark = pytest.mark.gpu
 
 
 # k padded to three and to four groups of 64; a last unit of 8 and of 40 features, a last token tile of 1 and of 6 tokens; t added up in ranges, their sums
-# ahead of N in the scratch; one token range of dC stored directly (the last case)
-@pytest.mark.parametrize("T,in_f,out_f,k", [(2817, 1416, 72, 136), (6000, 1000, 264, 200), (2824, 1416, 2120, 256), (16390, 264, 136, 144), (3000, 1608, 8, 256)])
+# ahead of N in the scratch; one token range of dC stored directly; rows of dx that are whole lines (1464 + 8 and 1976 + 8 features apart), with a last unit of 56
+# and a last token tile of 7 and of 8 tokens
+@pytest.mark.parametrize("T,in_f,out_f,k", [(2817, 1416, 72, 136), (6000, 1000, 264, 200), (2824, 1416, 2120, 256), (16390, 264, 136, 144), (3000, 1608, 8, 256),
+                                            (2823, 1464, 72, 192), (2824, 1976, 264, 256)])
 def test_from_memory_is_hashed_in_place(T, in_f, out_f, k):
     from randumb_amd import _lib, hip
 

@@ -56,9 +56,10 @@ def test_forward_against_float64(T, in_f, out_f, k):
 
 
 # both shares of dx and all gradients in one call: both kinds of tiles, k of one step, of no multiple of a step and the largest; the last case adds up dy . C
-# in ranges.  The scratch holds NaN beforehand; the first case's
-# state has no transposed coefficients
-@pytest.mark.parametrize("T,in_f,out_f,k", [(8100, 584, 72, 8), (5300, 1000, 136, 72), (16385, 200, 264, 200), (16264, 264, 72, 256), (2100, 2056, 2056, 72)])
+# in ranges; rows of dx that are whole lines (760 + 8 and 1016 + 8 features apart), which leave past the caches, in both kinds of tiles.  The scratch holds NaN
+# beforehand; the first case's state has no transposed coefficients
+@pytest.mark.parametrize("T,in_f,out_f,k", [(8100, 584, 72, 8), (5300, 1000, 136, 72), (16385, 200, 264, 200), (16264, 264, 72, 256), (2100, 2056, 2056, 72),
+                                            (8100, 760, 72, 72), (8190, 1016, 136, 200)])
 def test_backward_in_one_call_against_float64(T, in_f, out_f, k):
     from randumb_amd import _lib, hip
 

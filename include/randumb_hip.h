@@ -192,7 +192,8 @@ enum { RDB_OP_LINEAR_FWD = 0, RDB_OP_LINEAR_BWD_DX = 1, RDB_OP_LINEAR_BWD_DCOEF 
        RDB_OP_LINEAR_FWD_KEPT = 12, RDB_OP_LINEAR_BWD_PROJECTED_RBIAS = 13 };
 
 /* Device scratch (bytes) that entry point `op` can use for `desc`; 0 when it has no use for any.  A NULL or too small
- * workspace is never an error with RDB_ALGO_AUTO: the library then runs a kernel that needs none. */
+ * workspace is never an error with RDB_ALGO_AUTO: the library then runs a kernel that needs none.  Not so for the calls that say how much
+ * they need: rdb_linear_project_fwd_rbias and rdb_linear_bwd_projected_rbias refuse less (RDB_E_WORKSPACE), and a layer for which their amount is 0. */
 int64_t rdb_linear_workspace_bytes(int op, const rdb_linear_desc *desc);
 
 /* Replaces the dispatch of aten.mm / aten.addmm on a pseudorandom tensor: materialize() then the dense
@@ -425,7 +426,8 @@ int rdb_linear_bwd_projected_part(int part, void *dx, int64_t lddx, float *dcoef
  * 256-wide tiles with one persistent block per compute unit; all others on 128-wide tiles.  mode 0: never the 256-wide
  * kernels; 1 (default): by that rule; 2: whenever k > 256 (for tests on small layers).  Both kinds contract in the same
  * order: y and dx are the same bit for bit; dcoef is contracted over all tokens in one pass by the 256-wide kernels, where the
- * 128-wide ones may add partial sums over token ranges (same values up to fp32 rounding).  Process-wide; returns the previous
+ * 128-wide ones may add partial sums over token ranges (same values up to fp32 rounding).  The products with a fused random bias follow the same mode,
+ * whatever k: mode 0 adds its share to a y or dx that was rounded before, where 1 and 2 may form both shares in one product.  Process-wide; returns the previous
  * mode. */
 int rdb_set_big_tiles(int mode);
 

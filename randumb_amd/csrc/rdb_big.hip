@@ -427,11 +427,12 @@ __global__ __launch_bounds__(256, 1) void big_z_kernel(BigZParams p)
 }
 
 // ----------------------------------------------------------------------------------------------- out += s * src . R^T (or R)
-// The fused random bias's share (rdb_rbias.hip) with R written once as bf16 and read back.  Hashed into the product it costs its hash
-// for every 512 tokens on tiles of 64 features: 75 us for 38.6 GFLOP in either direction at 8192 tokens x 768 -> 3072; here 63 forward
-// (three tiles a block, each with 128 KB of dst to read and write) and 50 backward (one tile of 48 stages a block), and 5 for R.  Tiles
-// of 256 features x 128 tokens, so that 768 features still give 192 of them, or 192 x 128 (rbias_big_rows); one persistent block a compute unit.  What the epilogue
-// adds to is requested before a tile's main loop, the next tile's first stages before its epilogue.
+// The fused random bias's share alone (rdb_rbias.hip) with R written once as bf16 and read back: layers that have no product of both shares
+// (backward with more than 256 coefficients, chunks of tokens) and calls for this share.  Hashed into the product it costs its hash for every 512 tokens
+// on tiles of 64 features: 63 us forward and 71 backward for 38.6 GFLOP at 8192 tokens x 768 -> 3072; here 52 forward (3072 features: 768 tiles of 256,
+// three a block, each with 64 KB of dst to read and to write) and 46 backward (768 features: 256 tiles of 192, one of 48 stages a block), and 5 to 7 for R.
+// Tiles of 256 features x 128 tokens or of 192 x 128 (rbias_big_rows); one persistent block a compute unit.  What the epilogue adds to is requested
+// before a tile's main loop, the next tile's first stages before its epilogue.
 struct BigRBiasParams {
     const bf16_t *noise;    // [cols x contraction] in fragment order
     const bf16_t *src;      // [tokens x contraction]
@@ -637,9 +638,11 @@ template <bool BIAS> __global__ __launch_bounds__(256, 1) void big_yr_kernel(Big
 // ----------------------------------------------------------------------------------------------- dx = t . N + s * dy . R
 // The backward pass of a layer with a fused random bias, second launch: a tile contracts dy with R, its sums times x are its share of the scale's
 // gradient; scaled by s they go on with t and N, so that dx is written once, rounded once, and never read back, and N, written down by the launch
-// before like R, is not hashed once a row tile.  Blocks behind the tiles' add up the coefficient gradient's token ranges.  Bound by the matrix cores
-// and the chip's power, like big_rbias_kernel, whose tiles these are; x is read as the accumulators lie, half a cache line a piece, all of it on its
-// way before the main loop.  us of the layer's step with the random bias in launches of its own (the table, dx +=) and with this: 8192 tokens x
+// before like R, is not hashed once a row tile.  Blocks behind the tiles' add up the coefficient gradient's token ranges: they take a tile's
+// registers, one wave a SIMD, and start where a tile is done or a unit has none.  41.9 GFLOP at 8192 tokens x 768 -> 3072, k = 256, 256 tiles for 256 units: 51 us
+// by itself, 46 (0.91 PFLOP/s) without those sums, 50 to 64 within a step; 4096 x 1536 -> 4096, k = 128: 56 and 54; 8192 x 1024 -> 2048, k = 256: 45 and 43.
+// A tile is big_rbias_kernel's.  Where the rest goes above the 36 us of the best large products is not measured: with one tile a block nothing
+// covers its start and its epilogue.  x is read as the accumulators lie, half a cache line a piece, all of it on its way before the main loop.  us of the layer's step with the random bias in launches of its own (the table, dx +=) and with this: 8192 tokens x
 // 768 -> 3072, k = 256: 165.6, 160.2; 4096 x 1536 -> 4096, k = 128: 173.5, 167.3; 8192 x 2048 -> 768, k = 64: 120.7, 111.3; 8192 x 1024 -> 2048,
 // k = 256: 146.8, 138.1; 5000 x 3072 -> 2000, k = 64: 212.1, 202.6; 4096 x 4096 -> 8192, k = 256: 724, 709; no size measured got slower, so all
 // layers take it whose t fits the launch's fragment order (k <= 256) and whose R is written to memory at all (rbias_big_table_bytes).
@@ -978,9 +981,11 @@ int64_t rbias_big_table_bytes(const rdb_linear_desc *d, int64_t cols, int num_cu
 }
 
 // Features of a tile of the product above: 192 where as many rounds of tiles as with 256 do, which are more tiles then, for compute units
-// that stood idle.  A round takes 0.93 of one with 256 features (the chip's power again), so another round is never worth it.  us of the step with
+// that stood idle.  A round takes 0.93 of one with 256 features, so another round is never worth it.  us of the step with
 // 256 and with 192 features a tile: 8192 tokens x 768 -> 3072, k = 256, 192 and 256 tiles 179.6, 176.2; 4096 x 1536 -> 4096, k = 128, the same
-// 186.6, 182.4; 8192 x 1024 -> 2048, 256 and 384: 152.9, 166.0; 5000 x 3072 -> 2000, 480 and 640: 222.2, 239.3.
+// 186.6, 182.4; 8192 x 1024 -> 2048, 256 and 384: 152.9, 166.0; 5000 x 3072 -> 2000, 480 and 640: 222.2, 239.3.  us of the forward share alone (y of the
+// second figure's features), the same: 8192 x 3072 -> 768, 192 and 256 tiles 52.2, 49.7; 4096 x 4096 -> 1536 65.9, 62.6; 12000 x 1024 -> 960, 376 and 470: 44.7,
+// 41.1; 16384 x 2048 -> 136, 128 of either: 34.4, 33.8; another round: 8192 x 768 -> 3072, 768 and 1024: 65.3, 71.0; 8192 x 2048 -> 1024, 256 and 384: 42.0, 61.4.
 static int rbias_big_rows(int64_t cols, int64_t tokens, int num_cus)
 {
     auto rounds = [&](int rows) { return cdiv(cdiv(cols, rows) * cdiv(tokens, BR_TOK), num_cus); };
@@ -1057,7 +1062,7 @@ int linear_fwd_rbias_big(void *y, int64_t ldy, const void *x, int64_t ldx, const
     return launch_big(big_yr_kernel<false>, p, p.tiles_o * p.tiles_t, num_cus, smem, s, "big_yr_kernel");
 }
 
-// dx = t . N + s * dy . R and the scale's gradient, from the tables of rbias_dx_table and noise_dx_table; red: NULL, or sums to be added up beside it
+// dx = t . N + s * dy . R and the scale's gradient, from the tables of rbias_dx_table and noise_dx_table; red: NULL, or sums to be added up behind its tiles
 int linear_dx_rbias_big(void *dx, int64_t lddx, const void *t, const void *dy, int64_t lddy, const RBiasDx &rb, const RedParams *red, const rdb_linear_desc *d,
                         int num_cus, hipStream_t s)
 {

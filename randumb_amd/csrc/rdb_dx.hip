@@ -472,7 +472,9 @@ int linear_dx_factored(void *dx, int64_t lddx, const void *dy, int64_t lddy, con
 static thread_local int g_bwd_parts = 3;
 void set_bwd_projected_parts(int mask) { g_bwd_parts = mask & 3; }
 
-// Blocks that write the tables, behind the others: short ones, so that every unit that is done with the products finds one.  us of the step with 32,
+// Blocks that write the tables, behind the others: short ones, so that every unit that is done with the products finds one.  They take a product's
+// registers and LDS and so run mostly as the launch's tail: what they save is launches and passes over memory, not the hash (34.4 us without tables and 39.8
+// with N and R, 2.6 M values, at 8192 tokens x 768 -> 3072, k = 256).  us of the step with 32,
 // 128, 512 and 1024 of them on 256 units: 8192 tokens x 768 -> 3072, k = 256: 176.4, 167.6, 164.8, 164.4; 4096 x 1536 -> 4096, k = 128: 197.5, 177.1,
 // 169.8, 170.0; 4096 x 4096 -> 8192, k = 256: 856, 727, 707, 717; 8192 x 2048 -> 768, k = 64: 116.8, 113.5, 113.4, 113.5.
 static int table_blocks(uint32_t pieces, int num_cus) { return (int)std::min<int64_t>(cdiv(pieces, 256), 2 * num_cus); }

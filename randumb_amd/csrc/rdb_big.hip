@@ -645,7 +645,8 @@ template <bool BIAS> __global__ __launch_bounds__(256, 1) void big_yr_kernel(Big
 // covers its start and its epilogue.  x is read as the accumulators lie, half a cache line a piece, all of it on its way before the main loop.  us of the layer's step with the random bias in launches of its own (the table, dx +=) and with this: 8192 tokens x
 // 768 -> 3072, k = 256: 165.6, 160.2; 4096 x 1536 -> 4096, k = 128: 173.5, 167.3; 8192 x 2048 -> 768, k = 64: 120.7, 111.3; 8192 x 1024 -> 2048,
 // k = 256: 146.8, 138.1; 5000 x 3072 -> 2000, k = 64: 212.1, 202.6; 4096 x 4096 -> 8192, k = 256: 724, 709; no size measured got slower, so all
-// layers take it whose t fits the launch's fragment order (k <= 256) and whose R is written to memory at all (rbias_big_table_bytes).
+// layers take it whose t the first launch leaves in fragment order (k <= 256; for the row-major t of longer contractions it is not built) and whose R is
+// written to memory at all (rbias_big_table_bytes).
 struct BigDxParams {
     const bf16_t *r, *n;    // R [in_f x out_f] and N^T [in_f x k], fragment order
     const bf16_t *dy;       // [tokens x out_f]

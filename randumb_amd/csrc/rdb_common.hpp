@@ -42,32 +42,57 @@ __device__ __forceinline__ uint32_t sq5_tail(uint32_t b)
     return b;
 }
 
-// The same for kernels that do nothing but hash, with six waves a SIMD or more.  An exclusive or that the compiler cannot merge with the
-// addition that follows: v_xad_u32 occupies the vector ALU longer than v_xor_b32 and v_add_u32 together when other waves' instructions
-// are there to issue beside those (4.4 against 2 x 2.6 clocks a wave; a hash and its use: 2.79 -> 3.03 T/s).  In the kernels that
-// hash between matrix instructions, with two waves a SIMD, the merged form is the faster one (8192 x 768 -> 3072 random-bias shares: 3 %).
-__device__ __forceinline__ uint32_t sq5_xor(uint32_t a, uint32_t b)
+// The same, four values at a time and written out, for kernels that do nothing but hash.  Two waves of a SIMD can have a vector instruction issued in
+// the same four clocks, but only two of the simple kind (shift, exclusive or, addition: 2.05 clocks each then).  A product, a conversion, a matrix
+// instruction, v_xad_u32 go alone, and the older wave goes first: while it has a vector instruction in every slot, the younger one stands at
+// its first product until the older has left the loop, and nothing is issued together (54 clocks a hash for its 14 instructions, with 8, 4 and 2 waves a
+// SIMD alike).  So those that go alone come in groups, and a wave at a group has the higher priority: the other one loses the slots of the group and no more.
+// A hash, its conversion and its multiply-add: 56 -> 42 clocks, waits for LDS included.  (An s_nop on either side of every such instruction opens
+// the slots too, 43 clocks, but only for waves in step: with LDS reads between 47 to 50.)
+#define SQ5_SHIFTS(H, T, A, ADD, B)                                                                                      \
+    "v_lshrrev_b32 " T ", " A ", " H "\n\tv_xor_b32 " H ", " T ", " H "\n\tv_add_u32 " H ", " ADD ", " H "\n\t"            \
+    "v_lshrrev_b32 " T ", " B ", " H "\n\tv_xor_b32 " H ", " T ", " H "\n\t"
+#define SQ5_FIRST(I0, I1, I2, I3) "s_setprio 1\n\t" I0 "\n\t" I1 "\n\t" I2 "\n\t" I3 "\n\ts_setprio 0\n\t"
+#define SQ5_MUL(H, N) "v_mul_lo_u32 " H ", " H ", " N
+// operands 0 .. 3 in place, from the first round's values up to the last product; T a scratch register, N3 and N5 the multipliers
+#define SQ5_FOUR(T, N3, N5)                                                                                              \
+    SQ5_SHIFTS("%0", T, "9", "0xa884f197", "11") SQ5_SHIFTS("%1", T, "9", "0xa884f197", "11")                            \
+    SQ5_SHIFTS("%2", T, "9", "0xa884f197", "11") SQ5_SHIFTS("%3", T, "9", "0xa884f197", "11")                            \
+    SQ5_FIRST(SQ5_MUL("%0", N3), SQ5_MUL("%1", N3), SQ5_MUL("%2", N3), SQ5_MUL("%3", N3))                                \
+    SQ5_SHIFTS("%0", T, "13", "0xb79f3abb", "15") SQ5_SHIFTS("%1", T, "13", "0xb79f3abb", "15")                          \
+    SQ5_SHIFTS("%2", T, "13", "0xb79f3abb", "15") SQ5_SHIFTS("%3", T, "13", "0xb79f3abb", "15")                          \
+    SQ5_FIRST(SQ5_MUL("%0", N5), SQ5_MUL("%1", N5), SQ5_MUL("%2", N5), SQ5_MUL("%3", N5))
+static_assert(SQ5_N2 == 0xa884f197u && SQ5_N4 == 0xb79f3abbu, "the additions of SQ5_FOUR");
+
+// sum += c[i] 2^31 noise(first + i N1), i = 0 .. 3, one fused multiply-add after the other; first += 4 N1
+__device__ __forceinline__ void sq5_four_terms(uint32_t &first, float &sum, const float __attribute__((ext_vector_type(4))) &c)
 {
-    uint32_t r;
-    asm("v_xor_b32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
+    uint32_t h[4], t;
+    asm("v_mov_b32 %0, %5\n\tv_add_u32 %1, 0xd2a80a3f, %5\n\tv_add_u32 %2, 0xa550147e, %5\n\tv_add_u32 %3, 0x77f81ebd, %5\n\t"
+        SQ5_FOUR("%4", "%7", "%8")
+        "v_lshrrev_b32 %4, 17, %0\n\tv_xor_b32 %0, %4, %0\n\tv_lshrrev_b32 %4, 17, %1\n\tv_xor_b32 %1, %4, %1\n\t"
+        "v_lshrrev_b32 %4, 17, %2\n\tv_xor_b32 %2, %4, %2\n\tv_lshrrev_b32 %4, 17, %3\n\tv_xor_b32 %3, %4, %3\n\t"
+        SQ5_FIRST("v_cvt_f32_i32 %0, %0", "v_cvt_f32_i32 %1, %1", "v_cvt_f32_i32 %2, %2", "v_cvt_f32_i32 %3, %3")
+        "v_add_u32 %5, 0x4aa028fc, %5\n\t"
+        "v_fmac_f32 %6, %0, %9\n\tv_fmac_f32 %6, %1, %10\n\tv_fmac_f32 %6, %2, %11\n\tv_fmac_f32 %6, %3, %12"
+        : "=&v"(h[0]), "=&v"(h[1]), "=&v"(h[2]), "=&v"(h[3]), "=&v"(t), "+v"(first), "+v"(sum)
+        : "s"(SQ5_N3), "s"(SQ5_N5), "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]));
 }
-// ... up to the last round's shift
-__device__ __forceinline__ uint32_t sq5_tail_apart_but_last(uint32_t b)
+static_assert(SQ5_N1 == 0xd2a80a3fu && 2u * SQ5_N1 == 0xa550147eu && 3u * SQ5_N1 == 0x77f81ebdu && 4u * SQ5_N1 == 0x4aa028fcu, "the additions of sq5_four_terms");
+
+// h[i] = the hash of the first-round value f[i] + m, exclusive-or mask (in a vector register), for a matrix instruction that follows: it has the higher
+// priority too, which the next call, or the kernel, takes back.  (The s_nop: two instructions have to lie between a vector instruction and a
+// matrix instruction that reads its result.)
+__device__ __forceinline__ void sq5_four_masked(const int __attribute__((ext_vector_type(4))) &f, uint32_t m, uint32_t mask, uint32_t (&h)[4])
 {
-    b = sq5_xor(b, b >> 9);
-    b += SQ5_N2;
-    b ^= (b >> 11);
-    b *= SQ5_N3;
-    b = sq5_xor(b, b >> 13);
-    b += SQ5_N4;
-    b ^= (b >> 15);
-    return b * SQ5_N5;
-}
-__device__ __forceinline__ uint32_t sq5_tail_apart(uint32_t b)
-{
-    b = sq5_tail_apart_but_last(b);
-    return b ^ (b >> 17);
+    uint32_t t;
+    asm("s_setprio 0\n\tv_add_u32 %0, %5, %9\n\tv_add_u32 %1, %6, %9\n\tv_add_u32 %2, %7, %9\n\tv_add_u32 %3, %8, %9\n\t"
+        SQ5_FOUR("%4", "%11", "%12")
+        "v_lshrrev_b32 %4, 17, %0\n\tv_bitop3_b32 %0, %4, %0, %10 bitop3:0x96\n\tv_lshrrev_b32 %4, 17, %1\n\tv_bitop3_b32 %1, %4, %1, %10 bitop3:0x96\n\t"
+        "v_lshrrev_b32 %4, 17, %2\n\tv_bitop3_b32 %2, %4, %2, %10 bitop3:0x96\n\tv_lshrrev_b32 %4, 17, %3\n\tv_bitop3_b32 %3, %4, %3, %10 bitop3:0x96\n\t"
+        "s_setprio 1\n\ts_nop 0"
+        : "=&v"(h[0]), "=&v"(h[1]), "=&v"(h[2]), "=&v"(h[3]), "=&v"(t)
+        : "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(m), "v"(mask), "s"(SQ5_N3), "s"(SQ5_N5));
 }
 
 __device__ __forceinline__ uint32_t sq5_bits(uint32_t idx, uint32_t seed) { return sq5_tail(idx * SQ5_N1 + seed); }

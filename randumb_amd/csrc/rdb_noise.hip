@@ -46,21 +46,19 @@ __global__ __launch_bounds__(NT) void sq5_fill_1d_kernel(float *__restrict__ out
 // order the reference's CUDA kernel uses, rten.cu:101-104).  Bound by the hash on the vector ALU.
 // GATHER = false: a = (n % Q)*sQ + (n / Q)*sP                       (RandumbTensor.py:264)
 // GATHER = true : a = idx[n / Q]*Q + n % Q   (Q = rowsize)          (RandumbTensor.py:1029)
-// A thread's terms are one chain of dependent instructions, on purpose: eight waves a SIMD fill each other's gaps, and two waves'
-// instructions can issue together where one wave's cannot (several elements a thread, or their terms interleaved: 2.6 - 2.8
-// Thash/s; this form: 3.0 at 768 x 3072 elements, k = 256, 222 -> 200 us, 3.1 at k = 1024).  Also measured: the terms as bytes of an 8-bit
-// matrix operand, without conversion and multiplication on the vector ALU (v_mfma_i32_16x16x64_i8): 229 us.
+// A thread's terms are one chain, four of them hashed side by side, in the order of instructions that lets two waves issue together (sq5_four_terms):
+// 768 x 3072 elements, k = 256: 218 -> 195 us; 524288 elements, k = 4096: 686 -> 590 (3.64 Thash/s; one term after the other, as the compiler orders it, 3.13).
+// Also measured, before that: the terms as bytes of an 8-bit matrix operand, without conversion and multiplication on the vector ALU
+// (v_mfma_i32_16x16x64_i8): 229 us.
 constexpr int COEF_CHUNK = 2048;
 // Coefficients below this in magnitude: 2^31 times their terms stays finite, and so do sums of them; others (and NaNs) get the factor 2^-31
-// term by term.  Without it, and with MAT_UNROLL terms a turn of the loop (still one after the other), a term takes 17 vector instructions
-// instead of 19: 768 x 3072 elements, k = 256: 219 -> 205 us, and the pass of that layer, 1024 tokens, 538 -> 520 (another box: 558 -> 550); 4096 rows of a 50304 x
-// 768 table, forward and backward, 525 -> 522 (one term a turn: 540).  The round constants stay literals: in scalar or vector registers the
-// same instructions take 2 to 6 % longer.  What is left of a chunk goes by fours and twos.  The look at the coefficients costs a launch about
+// term by term.  Without it a term takes two vector instructions less.  A turn of the loop is MAT_UNROLL terms, whose coefficients were read the turn before (turns of
+// 8: 43.2 clocks a hash, of 16: 42.2).  What is left of a chunk goes by fours.  The look at the coefficients costs a launch about
 // a microsecond, which up to MAT_SHORT terms are not paid back: those get the factor term by term.  768 x 3072 elements, term by term
 // and otherwise: k = 8 11.8 and 13.9 us, 23 22.9 and 24.5, 48 41.2 and 42.1, 64 52.9 and 53.6, 96 76.6 and 76.5, 256 194 and 190; 300 x 800
 // elements: 48 8.5 both, 64 9.1 and 8.7.
 constexpr float MAT_LARGE = 3.777893186295716e22f;   // 2^75
-constexpr int MAT_UNROLL = 8;
+constexpr int MAT_UNROLL = 16;
 constexpr int MAT_SHORT = 48;
 constexpr int64_t MAT_PAIR_HASHES = (int64_t)1 << 27;   // a weight and its bias in one launch: up to some 45 us of hashing
 
@@ -101,7 +99,7 @@ template <bool GATHER, int LANES, bool SHORT> __device__ __forceinline__ void ma
         if (SHORT || __syncthreads_or(large)) {
             if (live)
                 for (int j = part; j < cnt; j += LANES) {
-                    acc = fmaf(sq5_unit(sq5_tail_apart(first)), cs[j], acc);
+                    acc = fmaf(sq5_unit(sq5_tail(first)), cs[j], acc);
                     first += LANES * SQ5_N1;
                 }
             continue;
@@ -110,26 +108,28 @@ template <bool GATHER, int LANES, bool SHORT> __device__ __forceinline__ void ma
             // 2^31 times the sum: the terms' common factor is taken out of the loop (a power of two: the same roundings)
             float sum = acc * 2147483648.0f;
             int j = part;
-            if (LANES == 1) {
-                auto turn = [&](auto terms) __attribute__((always_inline)) {
-                    constexpr int TERMS = decltype(terms)::value;
-                    float c[TERMS];
+            if (LANES == 1 && cnt >= MAT_UNROLL) {
+                // coefficients are read a turn ahead
+                uint32_t at = 0;
+                asm("" : "+v"(at));   // an address in a vector register: moving it there costs a slot a read
+                auto read = [&](int e) { return *reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(cs) + at + e * 4); };
+                f32x4 c[MAT_UNROLL / 4];
 #pragma unroll
-                    for (int e = 0; e < TERMS; ++e) c[e] = cs[j + e];
+                for (int q = 0; q < MAT_UNROLL / 4; ++q) c[q] = read(q * 4);
+                for (; j + MAT_UNROLL <= cnt; j += MAT_UNROLL) {
 #pragma unroll
-                    for (int e = 0; e < TERMS; ++e) {
-                        sum = fmaf((float)(int32_t)sq5_tail_apart(first), c[e], sum);
-                        first += SQ5_N1;
-                        __builtin_amdgcn_sched_barrier(0);   // one term after the other
+                    for (int q = 0; q < MAT_UNROLL / 4; ++q) {
+                        sq5_four_terms(first, sum, c[q]);
+                        c[q] = read(MAT_UNROLL + q * 4);
+                        __builtin_amdgcn_sched_barrier(0);
                     }
-                    j += TERMS;
-                };
-                while (j + MAT_UNROLL <= cnt) turn(std::integral_constant<int, MAT_UNROLL>{});
-                if (j + 4 <= cnt) turn(std::integral_constant<int, 4>{});
-                if (j + 2 <= cnt) turn(std::integral_constant<int, 2>{});
+                    at += MAT_UNROLL * 4;
+                }
             }
+            if (LANES == 1)
+                for (; j + 4 <= cnt; j += 4) sq5_four_terms(first, sum, *reinterpret_cast<const f32x4 *>(cs + j));
             for (; j < cnt; j += LANES) {
-                sum = fmaf((float)(int32_t)sq5_tail_apart(first), cs[j], sum);
+                sum = fmaf((float)(int32_t)sq5_tail(first), cs[j], sum);
                 first += LANES * SQ5_N1;
             }
             acc = sum * 4.656612873077392578125e-10f;
@@ -144,13 +144,13 @@ template <bool GATHER, int LANES, bool SHORT> __device__ __forceinline__ void ma
 }
 template <bool GATHER, int LANES, bool SHORT> __global__ __launch_bounds__(NT) void materialize_vec_kernel(MatVecParams p)
 {
-    __shared__ __align__(16) float cs[COEF_CHUNK];
+    __shared__ __align__(16) float cs[COEF_CHUNK + MAT_UNROLL];   // reads run a turn ahead
     materialize_vec_block<GATHER, LANES, SHORT>(p, cs, blockIdx.x);
 }
 // A weight and its bias, contiguous both: the bias's blocks (16 lanes an element) first.
 template <int LANES, bool SHORT> __global__ __launch_bounds__(NT) void materialize_vec_pair_kernel(MatVecParams weight, MatVecParams bias, unsigned bias_blocks)
 {
-    __shared__ __align__(16) float cs[COEF_CHUNK];
+    __shared__ __align__(16) float cs[COEF_CHUNK + MAT_UNROLL];   // reads run a turn ahead
     if (blockIdx.x < bias_blocks) materialize_vec_block<false, 16, false>(bias, cs, blockIdx.x);
     else materialize_vec_block<false, LANES, SHORT>(weight, cs, blockIdx.x - bias_blocks);
 }
@@ -238,16 +238,11 @@ __global__ __launch_bounds__(NT) void materialize_mat_tiled_kernel(float *__rest
 // (element, byte).  The 32-bit sums are exact for up to 2^14 elements; they are put together in fp64 and rounded once.  (Bytes 0 .. 2 of n
 // are unsigned where the instruction takes signed ones: n ^ 0x00808080 gives n - 128 (1 + 2^8 + 2^16), and 8421504 . sum q is
 // added back.)  13 vector instructions a term and no LDS read: 768 x 3072 elements, k = 256: 250 -> 204 us (2.95 Thash/s), and
-// 33 -> 4 for the partial rows' sum.
+// 33 -> 4 for the partial rows' sum; with the order of instructions of sq5_four_masked and the operands of a step read ahead 214 -> 191, 16 M elements
+// 1453 -> 1252 (3.43 Thash/s).
 typedef int q8x4 __attribute__((ext_vector_type(4)));
 constexpr double Q_OFFSET = 8421504.0;   // 128 (1 + 2^8 + 2^16)
-
-// b: first-round value
-__device__ __forceinline__ int q8_hash(uint32_t b)
-{
-    b = sq5_tail_apart_but_last(b);
-    return (int)__builtin_amdgcn_bitop3_b32(b, b >> 17, 0x00808080u, 0x96);   // three-way exclusive or in one instruction
-}
+constexpr uint32_t Q_MASK = 0x00808080u;
 
 // p with which values of at most the magnitude behind `top` (the largest |v| as bits, finite), times 2^p, stay below 2^38
 __device__ __forceinline__ int q8_exponent(uint32_t top)
@@ -367,6 +362,8 @@ template <bool GATHER, int MT, int WM> __global__ __launch_bounds__(NT) void coe
         mterm[i] = (uint32_t)(m0 + i * 16) * SQ5_N1 + p.seed;
     }
     long long q = 0;
+    uint32_t mask = Q_MASK;
+    asm("" : "+v"(mask));   // stays in a vector register
     for (int64_t e0 = e_begin; e0 < e_end; e0 += NT) {
         const int64_t e = e0 + t;
         float dv = 0.0f;   // zero beyond the span, so the tail adds nothing
@@ -383,17 +380,35 @@ template <bool GATHER, int MT, int WM> __global__ __launch_bounds__(NT) void coe
         for (int s = 0; s < 8; ++s) win[s][t] = w[s];
         __syncthreads();
         const int steps = (int)((e_end - e0 < NT ? e_end - e0 : NT) + 15) / 16;
-        for (int st = wave / WM; st < steps; st += WE) {
-            const q8x4 d = *reinterpret_cast<const q8x4 *>(&win[lane & 7][st * 16 + grp * 4]);
-            const q8x4 f = *reinterpret_cast<const q8x4 *>(&as[st * 16 + grp * 4]);
+        // a step's operands are read while the one before is hashed
+        auto read = [&](int st, q8x4 &d, q8x4 &f) __attribute__((always_inline)) {
+            st = min(st, NT / 16 - 1);
+            d = *reinterpret_cast<const q8x4 *>(&win[lane & 7][st * 16 + grp * 4]);
+            f = *reinterpret_cast<const q8x4 *>(&as[st * 16 + grp * 4]);
+        };
+        auto step = [&](const q8x4 &d, const q8x4 &f) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
-                const q8x4 h = {q8_hash((uint32_t)f[0] + mterm[i]), q8_hash((uint32_t)f[1] + mterm[i]), q8_hash((uint32_t)f[2] + mterm[i]),
-                                q8_hash((uint32_t)f[3] + mterm[i])};
-                acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(d, h, acc[i], 0, 0, 0);
+                uint32_t h[4];
+                sq5_four_masked(f, mterm[i], mask, h);
+                acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(d, q8x4{(int)h[0], (int)h[1], (int)h[2], (int)h[3]}, acc[i], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
             }
+        };
+        q8x4 d0, f0, d1, f1;
+        int st = wave / WM;
+        read(st, d0, f0);
+        for (; st < steps; st += 2 * WE) {
+            read(st + WE, d1, f1);
+            __builtin_amdgcn_sched_barrier(0);
+            step(d0, f0);
+            if (st + WE >= steps) break;
+            read(st + 2 * WE, d0, f0);
+            __builtin_amdgcn_sched_barrier(0);
+            step(d1, f1);
         }
     }
+    __builtin_amdgcn_s_setprio(0);
     double offset = block_sum_ll(q, sums) * Q_OFFSET;
     if (wave / WM) offset = 0.0;   // once per block
 #pragma unroll

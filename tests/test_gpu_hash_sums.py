@@ -121,3 +121,16 @@ def test_few_terms_and_more(hip, n, k):
     got = hip.materialize_fwd(c, (n,), (1,), 11, None, False)
     # k fp32 multiply-adds one after the other, each rounded by at most 2^-24 of the running sum
     assert float((got.double() - noise @ c.double()).abs().max()) <= k * 2.0**-24 * float((noise.abs() @ c.double().abs()).max())
+
+
+@pytest.mark.parametrize("n,k", [(131073, 49), (131200, 63), (131073, 64), (140001, 67), (131100, 2047), (131073, 2065), (131073, 2115)])
+def test_one_thread_an_element_whatever_is_left_of_a_turn(hip, n, k):
+    """From 2^17 elements on: turns of 16 terms, then fours, then single ones, in each chunk of 2048."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    c, d = torch.randn(k, generator=g, device="cuda"), torch.randn(n, generator=g, device="cuda")
+    rows = torch.cat([torch.arange(300), torch.arange(n - 300, n)]).cuda()
+    noise = hip.sq5_fill_2d(n, k, 5)
+    # fp32 chains of k terms: 2^-24 each, relative to the largest partial sum
+    assert rel(hip.materialize_fwd(c, (n,), (1,), 5, None, False)[rows], noise[rows].double() @ c.double()) < 2e-6
+    want = sum(d[i : i + 20000].double() @ noise[i : i + 20000].double() for i in range(0, n, 20000))
+    assert rel(hip.materialize_bwd(d, k, 5), want) < 2e-6

@@ -54,14 +54,14 @@ __device__ __forceinline__ uint32_t sq5_tail(uint32_t b)
     "v_lshrrev_b32 " T ", " B ", " H "\n\tv_xor_b32 " H ", " T ", " H "\n\t"
 #define SQ5_FIRST(I0, I1, I2, I3) "s_setprio 1\n\t" I0 "\n\t" I1 "\n\t" I2 "\n\t" I3 "\n\ts_setprio 0\n\t"
 #define SQ5_MUL(H, N) "v_mul_lo_u32 " H ", " H ", " N
-// operands 0 .. 3 in place, from the first round's values up to the last product; T a scratch register, N3 and N5 the multipliers
-#define SQ5_FOUR(T, N3, N5)                                                                                              \
-    SQ5_SHIFTS("%0", T, "9", "0xa884f197", "11") SQ5_SHIFTS("%1", T, "9", "0xa884f197", "11")                            \
-    SQ5_SHIFTS("%2", T, "9", "0xa884f197", "11") SQ5_SHIFTS("%3", T, "9", "0xa884f197", "11")                            \
-    SQ5_FIRST(SQ5_MUL("%0", N3), SQ5_MUL("%1", N3), SQ5_MUL("%2", N3), SQ5_MUL("%3", N3))                                \
-    SQ5_SHIFTS("%0", T, "13", "0xb79f3abb", "15") SQ5_SHIFTS("%1", T, "13", "0xb79f3abb", "15")                          \
-    SQ5_SHIFTS("%2", T, "13", "0xb79f3abb", "15") SQ5_SHIFTS("%3", T, "13", "0xb79f3abb", "15")                          \
-    SQ5_FIRST(SQ5_MUL("%0", N5), SQ5_MUL("%1", N5), SQ5_MUL("%2", N5), SQ5_MUL("%3", N5))
+// four values in place, from the first round's up to the last product; T a scratch register, N3 and N5 the multipliers
+#define SQ5_FOUR(H0, H1, H2, H3, T, N3, N5)                                                                              \
+    SQ5_SHIFTS(H0, T, "9", "0xa884f197", "11") SQ5_SHIFTS(H1, T, "9", "0xa884f197", "11")                                \
+    SQ5_SHIFTS(H2, T, "9", "0xa884f197", "11") SQ5_SHIFTS(H3, T, "9", "0xa884f197", "11")                                \
+    SQ5_FIRST(SQ5_MUL(H0, N3), SQ5_MUL(H1, N3), SQ5_MUL(H2, N3), SQ5_MUL(H3, N3))                                        \
+    SQ5_SHIFTS(H0, T, "13", "0xb79f3abb", "15") SQ5_SHIFTS(H1, T, "13", "0xb79f3abb", "15")                              \
+    SQ5_SHIFTS(H2, T, "13", "0xb79f3abb", "15") SQ5_SHIFTS(H3, T, "13", "0xb79f3abb", "15")                              \
+    SQ5_FIRST(SQ5_MUL(H0, N5), SQ5_MUL(H1, N5), SQ5_MUL(H2, N5), SQ5_MUL(H3, N5))
 static_assert(SQ5_N2 == 0xa884f197u && SQ5_N4 == 0xb79f3abbu, "the additions of SQ5_FOUR");
 
 // sum += c[i] 2^31 noise(first + i N1), i = 0 .. 3, one fused multiply-add after the other; first += 4 N1
@@ -69,7 +69,7 @@ __device__ __forceinline__ void sq5_four_terms(uint32_t &first, float &sum, cons
 {
     uint32_t h[4], t;
     asm("v_mov_b32 %0, %5\n\tv_add_u32 %1, 0xd2a80a3f, %5\n\tv_add_u32 %2, 0xa550147e, %5\n\tv_add_u32 %3, 0x77f81ebd, %5\n\t"
-        SQ5_FOUR("%4", "%7", "%8")
+        SQ5_FOUR("%0", "%1", "%2", "%3", "%4", "%7", "%8")
         "v_lshrrev_b32 %4, 17, %0\n\tv_xor_b32 %0, %4, %0\n\tv_lshrrev_b32 %4, 17, %1\n\tv_xor_b32 %1, %4, %1\n\t"
         "v_lshrrev_b32 %4, 17, %2\n\tv_xor_b32 %2, %4, %2\n\tv_lshrrev_b32 %4, 17, %3\n\tv_xor_b32 %3, %4, %3\n\t"
         SQ5_FIRST("v_cvt_f32_i32 %0, %0", "v_cvt_f32_i32 %1, %1", "v_cvt_f32_i32 %2, %2", "v_cvt_f32_i32 %3, %3")
@@ -83,16 +83,22 @@ static_assert(SQ5_N1 == 0xd2a80a3fu && 2u * SQ5_N1 == 0xa550147eu && 3u * SQ5_N1
 // h[i] = the hash of the first-round value f[i] + m, exclusive-or mask (in a vector register), for a matrix instruction that follows: it has the higher
 // priority too, which the next call, or the kernel, takes back.  (The s_nop: two instructions have to lie between a vector instruction and a
 // matrix instruction that reads its result.)
-__device__ __forceinline__ void sq5_four_masked(const int __attribute__((ext_vector_type(4))) &f, uint32_t m, uint32_t mask, uint32_t (&h)[4])
+#define SQ5_MASKED(H, T, MASK) "v_lshrrev_b32 " T ", 17, " H "\n\tv_bitop3_b32 " H ", " T ", " H ", " MASK " bitop3:0x96\n\t"
+__device__ __forceinline__ void sq5_eight_masked(const int __attribute__((ext_vector_type(4))) &f, const int __attribute__((ext_vector_type(4))) &g, uint32_t m,
+                                                 uint32_t mask, int __attribute__((ext_vector_type(8))) &h)
 {
-    uint32_t t;
-    asm("s_setprio 0\n\tv_add_u32 %0, %5, %9\n\tv_add_u32 %1, %6, %9\n\tv_add_u32 %2, %7, %9\n\tv_add_u32 %3, %8, %9\n\t"
-        SQ5_FOUR("%4", "%11", "%12")
-        "v_lshrrev_b32 %4, 17, %0\n\tv_bitop3_b32 %0, %4, %0, %10 bitop3:0x96\n\tv_lshrrev_b32 %4, 17, %1\n\tv_bitop3_b32 %1, %4, %1, %10 bitop3:0x96\n\t"
-        "v_lshrrev_b32 %4, 17, %2\n\tv_bitop3_b32 %2, %4, %2, %10 bitop3:0x96\n\tv_lshrrev_b32 %4, 17, %3\n\tv_bitop3_b32 %3, %4, %3, %10 bitop3:0x96\n\t"
+    uint32_t t, v[8];
+    asm("s_setprio 0\n\tv_add_u32 %0, %9, %17\n\tv_add_u32 %1, %10, %17\n\tv_add_u32 %2, %11, %17\n\tv_add_u32 %3, %12, %17\n\t"
+        SQ5_FOUR("%0", "%1", "%2", "%3", "%8", "%19", "%20")
+        SQ5_MASKED("%0", "%8", "%18") SQ5_MASKED("%1", "%8", "%18") SQ5_MASKED("%2", "%8", "%18") SQ5_MASKED("%3", "%8", "%18")
+        "v_add_u32 %4, %13, %17\n\tv_add_u32 %5, %14, %17\n\tv_add_u32 %6, %15, %17\n\tv_add_u32 %7, %16, %17\n\t"
+        SQ5_FOUR("%4", "%5", "%6", "%7", "%8", "%19", "%20")
+        SQ5_MASKED("%4", "%8", "%18") SQ5_MASKED("%5", "%8", "%18") SQ5_MASKED("%6", "%8", "%18") SQ5_MASKED("%7", "%8", "%18")
         "s_setprio 1\n\ts_nop 0"
-        : "=&v"(h[0]), "=&v"(h[1]), "=&v"(h[2]), "=&v"(h[3]), "=&v"(t)
-        : "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(m), "v"(mask), "s"(SQ5_N3), "s"(SQ5_N5));
+        : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]), "=&v"(t)
+        : "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "v"(m), "v"(mask), "s"(SQ5_N3), "s"(SQ5_N5));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) h[i] = (int)v[i];
 }
 
 __device__ __forceinline__ uint32_t sq5_bits(uint32_t idx, uint32_t seed) { return sq5_tail(idx * SQ5_N1 + seed); }

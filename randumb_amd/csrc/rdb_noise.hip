@@ -6,6 +6,8 @@
 
 namespace rdb {
 
+int num_compute_units();   // rdb_error.hip
+
 constexpr int NT = 256;  // threads per block for every kernel in this file
 
 // =============================================================================================== probes
@@ -47,7 +49,7 @@ __global__ __launch_bounds__(NT) void sq5_fill_1d_kernel(float *__restrict__ out
 // GATHER = false: a = (n % Q)*sQ + (n / Q)*sP                       (RandumbTensor.py:264)
 // GATHER = true : a = idx[n / Q]*Q + n % Q   (Q = rowsize)          (RandumbTensor.py:1029)
 // A thread's terms are one chain, four of them hashed side by side, in the order of instructions that lets two waves issue together (sq5_four_terms):
-// 768 x 3072 elements, k = 256: 218 -> 195 us; 524288 elements, k = 4096: 686 -> 590 (3.64 Thash/s; one term after the other, as the compiler orders it, 3.13).
+// 768 x 3072 elements, k = 256: 189 -> 171 us; 524288 elements, k = 4096: 681 -> 590 (3.64 Thash/s; one term after the other, as the compiler orders it, 3.15).
 // Also measured, before that: the terms as bytes of an 8-bit matrix operand, without conversion and multiplication on the vector ALU
 // (v_mfma_i32_16x16x64_i8): 229 us.
 constexpr int COEF_CHUNK = 2048;
@@ -69,12 +71,15 @@ struct MatVecParams {
     int64_t k, Nw, Q, sP, sQ;
     int coef_dtype, narrow, contiguous;   // narrow: element numbers fit 32 bits; contiguous: element n has offset n
     uint32_t seed;
+    unsigned blocks;   // of NT / LANES elements
 };
 
 // LANES > 1: that many neighbouring lanes share an element, lane l its terms l, l + LANES, .. (then added up across the lanes, nearest
 // first): with few elements the chip is not full, and the chain's length is what a launch takes (3072 elements, k = 256: 16.5 ->
 // 4 us).  SHORT: at most MAT_SHORT terms.
-template <bool GATHER, int LANES, bool SHORT> __device__ __forceinline__ void materialize_vec_block(const MatVecParams &p, float *__restrict__ cs, unsigned block)
+// fill: the coefficients are not in cs yet, or do not fit all at once; one_factor: what a call that fills it says of them, for those that do not
+template <bool GATHER, int LANES, bool SHORT>
+__device__ __forceinline__ void materialize_vec_block(const MatVecParams &p, float *__restrict__ cs, unsigned block, bool fill, bool &one_factor)
 {
     const int64_t n = ((int64_t)block * NT + threadIdx.x) / LANES;
     const int part = threadIdx.x % LANES;
@@ -89,14 +94,17 @@ template <bool GATHER, int LANES, bool SHORT> __device__ __forceinline__ void ma
     int large = 0;   // stays so for the chunks that follow: the sum is large then
     for (int64_t m0 = 0; m0 < p.k; m0 += COEF_CHUNK) {   // a multiple of LANES
         const int cnt = (int)((p.k - m0) < COEF_CHUNK ? (p.k - m0) : COEF_CHUNK);
-        __syncthreads();
-        for (int j = threadIdx.x; j < cnt; j += NT) {
-            const float c = load_as_f32(p.coef, p.coef_dtype, m0 + j);
-            cs[j] = c;
-            large |= !(fabsf(c) < MAT_LARGE);
+        if (fill) {
+            __syncthreads();
+            for (int j = threadIdx.x; j < cnt; j += NT) {
+                const float c = load_as_f32(p.coef, p.coef_dtype, m0 + j);
+                cs[j] = c;
+                large |= !(fabsf(c) < MAT_LARGE);
+            }
+            if (SHORT) __syncthreads();
+            else one_factor = !__syncthreads_or(large);
         }
-        if (SHORT) __syncthreads();
-        if (SHORT || __syncthreads_or(large)) {
+        if (SHORT || !one_factor) {
             if (live)
                 for (int j = part; j < cnt; j += LANES) {
                     acc = fmaf(sq5_unit(sq5_tail(first)), cs[j], acc);
@@ -145,14 +153,17 @@ template <bool GATHER, int LANES, bool SHORT> __device__ __forceinline__ void ma
 template <bool GATHER, int LANES, bool SHORT> __global__ __launch_bounds__(NT) void materialize_vec_kernel(MatVecParams p)
 {
     __shared__ __align__(16) float cs[COEF_CHUNK + MAT_UNROLL];   // reads run a turn ahead
-    materialize_vec_block<GATHER, LANES, SHORT>(p, cs, blockIdx.x);
+    bool one_factor = false;
+    for (unsigned block = blockIdx.x; block < p.blocks; block += gridDim.x)
+        materialize_vec_block<GATHER, LANES, SHORT>(p, cs, block, block == blockIdx.x || p.k > COEF_CHUNK, one_factor);
 }
 // A weight and its bias, contiguous both: the bias's blocks (16 lanes an element) first.
 template <int LANES, bool SHORT> __global__ __launch_bounds__(NT) void materialize_vec_pair_kernel(MatVecParams weight, MatVecParams bias, unsigned bias_blocks)
 {
     __shared__ __align__(16) float cs[COEF_CHUNK + MAT_UNROLL];   // reads run a turn ahead
-    if (blockIdx.x < bias_blocks) materialize_vec_block<false, 16, false>(bias, cs, blockIdx.x);
-    else materialize_vec_block<false, LANES, SHORT>(weight, cs, blockIdx.x - bias_blocks);
+    bool one_factor = false;
+    if (blockIdx.x < bias_blocks) materialize_vec_block<false, 16, false>(bias, cs, blockIdx.x, true, one_factor);
+    else materialize_vec_block<false, LANES, SHORT>(weight, cs, blockIdx.x - bias_blocks, true, one_factor);
 }
 
 // Matrix-coef materialise, arbitrary view: one thread per output element (no sharing of noise between rows).
@@ -234,13 +245,15 @@ __global__ __launch_bounds__(NT) void materialize_mat_tiled_kernel(float *__rest
 // relative to the largest of the block's span (below 2^-39 of it is dropped; fp32 sums drop more at every addition), in five
 // signed base-256 digits, and
 //     sum n q = sum over s of 256^s . sum over (element, byte j of n) of byte_j(n) . digit_(s-j)(q)
-// is one v_mfma_i32_16x16x64_i8 per 16 elements x 16 coefficients: rows = s (0 .. 7, twice), columns = coefficients, contraction =
-// (element, byte).  The 32-bit sums are exact for up to 2^14 elements; they are put together in fp64 and rounded once.  (Bytes 0 .. 2 of n
+// is one matrix instruction per 32 elements x 16 coefficients: columns = coefficients, contraction = (element, byte), rows = s (0 .. 7) for
+// the lower two bytes of an element and again for the upper two.  Two of a row's four bytes an element are zeros then, always the same, so
+// it is the sparse one (v_smfmac_i32_16x16x128_i8), with twice the contraction of the dense one in the same time (16 M elements, k = 256: 1252 -> 1178 us).  The 32-bit sums are exact for up to 2^14 elements; they are put together in fp64 and rounded once.  (Bytes 0 .. 2 of n
 // are unsigned where the instruction takes signed ones: n ^ 0x00808080 gives n - 128 (1 + 2^8 + 2^16), and 8421504 . sum q is
 // added back.)  13 vector instructions a term and no LDS read: 768 x 3072 elements, k = 256: 250 -> 204 us (2.95 Thash/s), and
-// 33 -> 4 for the partial rows' sum; with the order of instructions of sq5_four_masked and the operands of a step read ahead 214 -> 191, 16 M elements
-// 1453 -> 1252 (3.43 Thash/s).
+// 33 -> 4 for the partial rows' sum; with the order of instructions of sq5_eight_masked, the operands of a step read ahead and those of the
+// next 256 elements fetched while these are hashed 208 -> 174 (3.47 Thash/s), 16 M elements 1449 -> 1190.
 typedef int q8x4 __attribute__((ext_vector_type(4)));
+typedef int q8x8 __attribute__((ext_vector_type(8)));
 constexpr double Q_OFFSET = 8421504.0;   // 128 (1 + 2^8 + 2^16)
 constexpr uint32_t Q_MASK = 0x00808080u;
 
@@ -270,14 +283,16 @@ __device__ __forceinline__ long long q8_windows(float v, double scale, uint32_t 
     return q;
 }
 
-// A result's rows are 4 (lane / 16) + j (r and r + 8 the same): put together.  Lanes 0 .. 31 take the columns of one accumulator, lanes
-// 32 .. 63 those of the other; the two halves of a column meet across 16 lanes.
+// A result's rows are 4 (lane / 16) + j; r and r + 8 belong together.  Lanes 0 .. 31 take the columns of one accumulator, lanes 32 .. 63 those of
+// the other; the two halves of a column meet across 16 lanes.
 __device__ __forceinline__ double q8_total(const q8x4 &low, const q8x4 &high)
 {
-    const bool second = threadIdx.x & 32;
     double v = 0.0;
 #pragma unroll
-    for (int j = 3; j >= 0; --j) v = v * 256.0 + (double)(second ? high[j] : low[j]);
+    for (int j = 3; j >= 0; --j) {
+        const auto s = __builtin_amdgcn_permlane32_swap((uint32_t)low[j], (uint32_t)high[j], false, false);
+        v = v * 256.0 + (double)(int)(s[0] + s[1]);
+    }
     if (threadIdx.x & 16) v *= 4294967296.0;
     const long long bits = __double_as_longlong(v);
     const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)bits, (uint32_t)bits, false, false);
@@ -330,8 +345,8 @@ template <bool GATHER> __device__ __forceinline__ uint32_t gradvec_offset(const 
 
 template <bool GATHER, int MT, int WM> __global__ __launch_bounds__(NT) void coef_grad_vec_kernel(GradVecParams p)
 {
-    constexpr int WE = 4 / WM, MBLOCK = 16 * MT * WM, LD = NT + 16;   // LD: eight rows apart in the banks by a quarter of them
-    __shared__ __align__(16) uint32_t win[8][LD];
+    constexpr int WE = 4 / WM, MBLOCK = 16 * MT * WM, LD = NT + 8;   // LD: 16 bytes of padding, so that 16 rows' pieces lie in different banks
+    __shared__ __align__(16) unsigned short win[16][LD];   // rows 0 .. 7: the windows' lower halves, 8 .. 15: their upper halves
     __shared__ __align__(16) uint32_t as[NT];
     __shared__ uint32_t tops[4];
     __shared__ long long sums[4];
@@ -364,48 +379,62 @@ template <bool GATHER, int MT, int WM> __global__ __launch_bounds__(NT) void coe
     long long q = 0;
     uint32_t mask = Q_MASK;
     asm("" : "+v"(mask));   // stays in a vector register
-    for (int64_t e0 = e_begin; e0 < e_end; e0 += NT) {
+    const int pairs = lane & 8 ? (int)0xeeeeeeeeu : 0x44444444;   // which two of an element's bytes this lane's row has: 2 and 3, or 0 and 1
+    float next_d;
+    uint32_t next_a;
+    auto fetch = [&](int64_t e0) {
         const int64_t e = e0 + t;
-        float dv = 0.0f;   // zero beyond the span, so the tail adds nothing
-        uint32_t a = 0;
+        next_d = 0.0f;   // zero beyond the span, so the tail adds nothing
+        next_a = 0;
         if (e < e_end) {
-            dv = load_as_f32(p.d, p.d_dtype, e);
-            a = gradvec_offset<GATHER>(p, e);
+            next_d = load_as_f32(p.d, p.d_dtype, e);
+            next_a = gradvec_offset<GATHER>(p, e);
         }
+    };
+    fetch(e_begin);
+    for (int64_t e0 = e_begin; e0 < e_end; e0 += NT) {
+        const float dv = next_d;
+        const uint32_t a = next_a;
+        fetch(e0 + NT);   // while this one is hashed
         uint32_t w[8];
         q += q8_windows(dv, scale, w);
         __syncthreads();
         as[t] = a * PN1;
 #pragma unroll
-        for (int s = 0; s < 8; ++s) win[s][t] = w[s];
+        for (int s = 0; s < 8; ++s) {
+            win[s][t] = (unsigned short)w[s];
+            win[s + 8][t] = (unsigned short)(w[s] >> 16);
+        }
         __syncthreads();
-        const int steps = (int)((e_end - e0 < NT ? e_end - e0 : NT) + 15) / 16;
-        // a step's operands are read while the one before is hashed
-        auto read = [&](int st, q8x4 &d, q8x4 &f) __attribute__((always_inline)) {
-            st = min(st, NT / 16 - 1);
-            d = *reinterpret_cast<const q8x4 *>(&win[lane & 7][st * 16 + grp * 4]);
-            f = *reinterpret_cast<const q8x4 *>(&as[st * 16 + grp * 4]);
+        const int steps = (int)((e_end - e0 < NT ? e_end - e0 : NT) + 31) / 32;
+        // A step is 32 elements: of the hashed operand, lane group g of a column has 4 g .. 4 g + 3 of each half of them; of the other one, lane group g of a
+        // row has 8 g .. 8 g + 7.  A step's operands are read while the one before is hashed.
+        auto read = [&](int st, q8x4 &d, q8x4 &f, q8x4 &g) __attribute__((always_inline)) {
+            st = min(st, NT / 32 - 1);
+            d = *reinterpret_cast<const q8x4 *>(&win[lane & 15][st * 32 + grp * 8]);
+            f = *reinterpret_cast<const q8x4 *>(&as[st * 32 + grp * 4]);
+            g = *reinterpret_cast<const q8x4 *>(&as[st * 32 + 16 + grp * 4]);
         };
-        auto step = [&](const q8x4 &d, const q8x4 &f) __attribute__((always_inline)) {
+        auto step = [&](const q8x4 &d, const q8x4 &f, const q8x4 &g) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
-                uint32_t h[4];
-                sq5_four_masked(f, mterm[i], mask, h);
-                acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(d, q8x4{(int)h[0], (int)h[1], (int)h[2], (int)h[3]}, acc[i], 0, 0, 0);
+                q8x8 h;
+                sq5_eight_masked(f, g, mterm[i], mask, h);
+                acc[i] = __builtin_amdgcn_smfmac_i32_16x16x128_i8(d, h, acc[i], pairs, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
-        q8x4 d0, f0, d1, f1;
+        q8x4 d0, f0, g0, d1, f1, g1;
         int st = wave / WM;
-        read(st, d0, f0);
+        read(st, d0, f0, g0);
         for (; st < steps; st += 2 * WE) {
-            read(st + WE, d1, f1);
+            read(st + WE, d1, f1, g1);
             __builtin_amdgcn_sched_barrier(0);
-            step(d0, f0);
+            step(d0, f0, g0);
             if (st + WE >= steps) break;
-            read(st + 2 * WE, d0, f0);
+            read(st + 2 * WE, d0, f0, g0);
             __builtin_amdgcn_sched_barrier(0);
-            step(d1, f1);
+            step(d1, f1, g1);
         }
     }
     __builtin_amdgcn_s_setprio(0);
@@ -518,11 +547,12 @@ static int grad_rows(int64_t k) { return k <= 16 ? 4 : k <= 32 ? 2 : 1; }
 // splits: partial rows in all
 static void split_plan(int64_t Nw, int64_t k, int64_t *splits, int64_t *span)
 {
-    // about six blocks a compute unit (24 waves), spans of a multiple of 256 elements and of at most 2^14
+    // about four blocks a compute unit (16 waves), of a multiple of 32 elements, 256 to 2^14 (six of a multiple of 256: 2.1 M elements, k = 256 174 -> 156 us, 0.8 M
+    // 77 -> 67; six of a multiple of 32: 160 and 70; three: 172 and 72; 2.4 M 174 each)
     const int64_t mblocks = cdiv(k, grad_block(k));
-    int64_t s = cdiv(Nw, NT), want = cdiv(1536, mblocks);
+    int64_t s = cdiv(Nw, NT), want = cdiv(1024, mblocks);
     if (s > want) s = want;
-    int64_t sp = cdiv(cdiv(Nw, s < 1 ? 1 : s), NT) * NT;
+    int64_t sp = cdiv(cdiv(Nw, s < 1 ? 1 : s), 32) * 32;
     if (sp < NT) sp = NT;
     if (sp > (1 << 14)) sp = 1 << 14;
     *span = sp;
@@ -534,9 +564,12 @@ static int mat_lanes(int64_t n, int64_t k) { return k < 8 ? 1 : n <= (1 << 15) ?
 static int launch_materialize_vec(float *out, const void *coef, int coef_dtype, int64_t k, int64_t Nw, int64_t Q, int64_t sP, int64_t sQ, uint32_t seed,
                                   const void *scale_bias, const int64_t *idx, hipStream_t s)
 {
-    const MatVecParams p = {out, coef, scale_bias, idx, k, Nw, Q, sP, sQ, coef_dtype, Nw < (1ll << 32) && Q < (1ll << 32), sQ == 1 && (sP == Q || Nw == Q), seed};
     const int lanes = mat_lanes(Nw, k);
-    const unsigned blocks = (unsigned)cdiv(Nw * lanes, NT);
+    const MatVecParams p = {out, coef, scale_bias, idx, k, Nw, Q, sP, sQ, coef_dtype, Nw < (1ll << 32) && Q < (1ll << 32), sQ == 1 && (sP == Q || Nw == Q), seed,
+                            (unsigned)cdiv(Nw * lanes, NT)};
+    // as many blocks as are resident at once, which take the elements in turns: their coefficients are read once, and no unit is left with a block more
+    // than others (blocks in turn -> so: 2.4 M elements, k = 256 173.7 -> 170.5 us; 0.8 M 65.6 -> 62.6; 1.5 M 113.6 -> 107.8; 2.9 M 215.0 -> 210.7; at most 0.5 M: even)
+    const unsigned blocks = std::min(p.blocks, 8u * (unsigned)num_compute_units());
     auto launch = [&](auto lanes_) {
         constexpr int L = decltype(lanes_)::value;
         auto run = [&](auto short_) {
@@ -650,7 +683,7 @@ extern "C" int rdb_materialize_weight_and_bias(float *weight, int64_t n, const f
     // Side by side where both are short; a long one's kernel stays as it is, and so do biases that get another number of lanes.
     if (n > 0 && bias_n > 0 && n * std::max<int64_t>(k, 1) <= MAT_PAIR_HASHES && mat_lanes(bias_n, bias->k) == 16) {
         const auto params = [](float *out, const float *c, const float *sc, int64_t terms, int64_t len, uint32_t sd) {
-            return MatVecParams{out, c, sc, nullptr, terms, len, len, 0, 1, RDB_F32, len < (1ll << 32), 1, sd};
+            return MatVecParams{out, c, sc, nullptr, terms, len, len, 0, 1, RDB_F32, len < (1ll << 32), 1, sd, 0};
         };
         const MatVecParams w = params(weight, coef, scale, k, n, seed), b = params(bias->values, bias->coef, bias->scale, bias->k, bias_n, bias->seed);
         const int lanes = mat_lanes(n, k);

@@ -134,3 +134,15 @@ def test_one_thread_an_element_whatever_is_left_of_a_turn(hip, n, k):
     assert rel(hip.materialize_fwd(c, (n,), (1,), 5, None, False)[rows], noise[rows].double() @ c.double()) < 2e-6
     want = sum(d[i : i + 20000].double() @ noise[i : i + 20000].double() for i in range(0, n, 20000))
     assert rel(hip.materialize_bwd(d, k, 5), want) < 2e-6
+
+
+@pytest.mark.parametrize("k", [16, 17, 40, 64, 100, 256])
+@pytest.mark.parametrize("n", [31, 32, 33, 255, 257, 287, 289, 600])
+def test_gradient_at_the_edges_of_a_step(hip, n, k):
+    """Steps of 32 elements, one to four waves along them, and values of one sign: every byte and digit counts."""
+    g = torch.Generator(device="cuda").manual_seed(n * 1000 + k)
+    d = torch.rand(n, generator=g, device="cuda") + 0.5
+    noise = hip.sq5_fill_2d(n, k, 6)
+    want = d.double() @ noise.double()
+    # integers throughout and one rounding of a sum of some sqrt(n), 6e-8 of it; the oracle's noise is rounded to fp32, 4.5e-8 a term at most, of either sign
+    assert float((hip.materialize_bwd(d, k, 6).double() - want).abs().max()) < 4e-7 * float(n) ** 0.5

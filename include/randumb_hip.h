@@ -83,9 +83,21 @@ int rdb_materialize_fwd(float *out, const void *coef, int coef_dtype, int64_t co
                         const void *scale_bias, void *stream);
 
 /* The weight (n values, contiguous) and the bias (bias_n values) of a vector-coef layer in fp32: what two calls of rdb_materialize_fwd
- * write, in one launch where the weight is small. */
+ * write, in one launch (biases of up to 2^15 values and 8 terms or more; two otherwise). */
 int rdb_materialize_weight_and_bias(float *weight, int64_t n, const float *coef, int64_t k, uint32_t seed, const float *scale,
                                     const rdb_pseudo_bias *bias, int64_t bias_n, void *stream);
+
+/* Backward pass of a vector-coef layer in fp32, y = x . W^T + b with W [out_f x in_f] and b formed by rdb_materialize_fwd: what two calls of
+ * rdb_product_f32 (dx = dy . W, dW = dy^T . x), rdb_materialize_bwd on dW and rdb_bias_bwd give, in four launches; dW is not kept.
+ *   dx         NULL, or [tokens x in_f], contiguous (W is read then)
+ *   dcoef      [k]
+ *   dbias_coef NULL, or [bias_k]: the gradient of a pseudorandom bias's coefficients
+ * RDB_E_UNSUPPORTED for empty sizes, matrices of 2^29 elements or more, and while fp32 products are asked for (rdb_set_f32_split); the query then
+ * returns 0.  Sums in fixed orders: results are bitwise reproducible run to run. */
+int64_t rdb_vector_linear_bwd_workspace_bytes(int64_t tokens, int64_t in_f, int64_t out_f, int64_t k, int want_dx, int want_bias);
+int rdb_vector_linear_bwd(float *dx, float *dcoef, float *dbias_coef, const float *dy, int64_t lddy, const float *x, int64_t ldx, const float *W,
+                          int64_t tokens, int64_t in_f, int64_t out_f, int64_t k, uint32_t seed, int64_t bias_k, uint32_t bias_seed,
+                          void *workspace, int64_t workspace_bytes, void *stream);
 
 /* Replaces: op rten::materialize_bwd + materialize_bwd_kernel (R.py:304-359, 383-390).
  * dW is a contiguous tensor of Nw elements (dtype dw_dtype).  dcoef is fp32 and is OVERWRITTEN:

@@ -33,6 +33,8 @@ EXPORTS = [
     "rdb_sq5_fill_1d",
     "rdb_materialize_fwd",
     "rdb_materialize_weight_and_bias",
+    "rdb_vector_linear_bwd",
+    "rdb_vector_linear_bwd_workspace_bytes",
     "rdb_materialize_bwd",
     "rdb_materialize_bwd_workspace_bytes",
     "rdb_scale_bias_bwd",
@@ -164,6 +166,10 @@ def load() -> ctypes.CDLL:
     L.rdb_sq5_fill_1d.argtypes = [vp, i64, u32, vp]
     L.rdb_materialize_weight_and_bias.argtypes = [vp, i64, vp, i64, u32, vp, vp, i64, vp]
     L.rdb_materialize_weight_and_bias.restype = ci
+    L.rdb_vector_linear_bwd.argtypes = [vp, vp, vp, vp, i64, vp, i64, vp, i64, i64, i64, i64, u32, i64, u32, vp, i64, vp]
+    L.rdb_vector_linear_bwd.restype = ci
+    L.rdb_vector_linear_bwd_workspace_bytes.argtypes = [i64, i64, i64, i64, ci, ci]
+    L.rdb_vector_linear_bwd_workspace_bytes.restype = i64
     L.rdb_materialize_fwd.argtypes = [vp, vp, ci, i64, i64, i64, i64, i64, i64, i64, u32, vp, vp]
     L.rdb_materialize_bwd.argtypes = [vp, vp, ci, i64, i64, i64, i64, u32, vp, i64, vp]
     L.rdb_materialize_bwd_workspace_bytes.argtypes = [i64, i64, i64, i64]

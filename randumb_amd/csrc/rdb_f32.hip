@@ -19,6 +19,7 @@
 // Replaces materialize() + dense product (src/rten_cpp/RandumbTensor.py:942-946) and MmBackward's dW followed by
 // materialize_bwd (RandumbTensor.py:979-990, 304-359) for fp32 layers beyond the few-token regime of rdb_smallk.hip.
 #include "rdb_f32.hpp"
+#include "rdb_sums.hpp"
 
 namespace rdb {
 
@@ -39,57 +40,11 @@ __global__ __launch_bounds__(256) void f32_sum_scalars_kernel(float *__restrict_
     if (threadIdx.x == 0) out[0] = sh[0];
 }
 
-// part[0] + part[stride] + ... in split order, eight loads in flight: one at a time the sum is a chain of `splits` memory latencies
-// (4097 tokens x 1001 -> 999 in bf16, k = 100: step 97 -> 91 us, three of these launches)
-template <typename V> __device__ __forceinline__ V sum_in_order(const float *__restrict__ part, int64_t stride, int splits)
-{
-    V v = *reinterpret_cast<const V *>(part);
-    for (int s0 = 1; s0 < splits; s0 += 8) {
-        V u[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) u[j] = *reinterpret_cast<const V *>(part + (int64_t)min(s0 + j, splits - 1) * stride);   // clamped: loaded, not added
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            if (s0 + j < splits) v += u[j];
-    }
-    return v;
-}
-
-// out[i] = part[0][i] + part[1][i] + ... in split order, four values per thread (n4 groups of four, then the n % 4 last values
-// one thread each); out fp32, or bf16 (rounded once); bias: NULL, or fp32, added to rows of cols values.  One or two such sums a launch:
-// the second one's blocks follow.
-struct FgSum {
-    void *out;
-    const float *part;
-    int64_t n, stride;   // values, floats between the partial matrices
-    int out_bf16, splits, vec;
-    int blocks;          // 0: no such sum
-    const float *bias;
-    uint32_t cols;
-};
+// One or two sums a launch: the second one's blocks follow.
 __global__ __launch_bounds__(256) void f32_sum_splits_kernel(FgSum a, FgSum b)
 {
     const bool second = (int)blockIdx.x >= a.blocks;
-    const FgSum &q = second ? b : a;
-    const int64_t i = (int64_t)((int)blockIdx.x - (second ? a.blocks : 0)) * 256 + threadIdx.x, n4 = q.vec ? q.n / 4 : 0;
-    if (i < n4) {
-        f32x4 v = sum_in_order<f32x4>(q.part + i * 4, q.stride, q.splits);
-        if (q.bias) {
-            uint32_t c = (uint32_t)(i * 4) % q.cols;   // n is below 2^29
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                v[j] += q.bias[c];
-                if (++c == q.cols) c = 0;
-            }
-        }
-        if (q.out_bf16) store4<bf16_t>(static_cast<bf16_t *>(q.out) + i * 4, v[0], v[1], v[2], v[3]);
-        else *reinterpret_cast<f32x4 *>(static_cast<float *>(q.out) + i * 4) = v;
-    } else if (n4 * 4 + (i - n4) < q.n) {
-        const int64_t e = n4 * 4 + (i - n4);
-        const float v = sum_in_order<float>(q.part + e, q.stride, q.splits) + (q.bias ? q.bias[(uint32_t)e % q.cols] : 0.0f);
-        if (q.out_bf16) static_cast<bf16_t *>(q.out)[e] = f32_to_bf16(v);
-        else static_cast<float *>(q.out)[e] = v;
-    }
+    f32_sum_block(second ? b : a, (int)blockIdx.x - (second ? a.blocks : 0));
 }
 static FgSum fg_sum(void *out, int out_bf16, const float *part, int64_t n, int64_t stride, int splits, const float *bias = nullptr, int64_t cols = 0)
 {
@@ -725,6 +680,72 @@ int coef_grad_mat_f32(float *dcoef, const void *dW, int dw_dtype, int64_t coef_r
 // ranges of 64 values and more: 216 tokens x 966 -> 198 took 30 us in one, 14 with the sums; dW of 497 tokens x 797 -> 410 22 -> 15
 static int product_room(int64_t M, int64_t N, int64_t K, int num_cus) { return fg_room(M, N, K, num_cus, 64, 64).ranges; }
 static bool product_ok(int64_t M, int64_t N, int64_t K) { return M > 0 && N > 0 && K > 0 && M * N < (1ll << 29) && K < (1 << 30); }
+
+// The products of a vector-coef layer's backward pass, dx = dy . W and dW = dy^T . x, side by side in one launch where both are wanted; what is left to
+// add up is left to a launch that comes anyway: dx's ranges (dx_sum, blocks 0: there are none), and dW's, as partial matrices (dw).
+static bool vector_products_ok(int64_t tokens, int64_t in_f, int64_t out_f)
+{
+    return product_ok(tokens, in_f, out_f) && product_ok(out_f, in_f, tokens) && tokens * out_f < (1ll << 29) && tokens * in_f < (1ll << 29) && f32_split_mode();
+}
+// dW's ranges: its partial matrices are added up where dW is contracted with the noise, which is the vector ALU's, so they cost memory traffic and its power: at most 16 MB
+// of them.  Vector-coef steps, us, with one, two, four, eight ranges at most: 1024 tokens x 512 -> 1024, k = 200 130, 118, 117, 118; 1500 x 300 -> 3000, k = 60 146,
+// 147, 130, 131; 2048 x 1024 -> 1024, k = 256 256, 245, 245, 244; 1024 x 768 -> 3072, k = 256, kept up for a second: 464, 475, 475, 477.
+static int vector_dw_room(int64_t tokens, int64_t in_f, int64_t out_f, int num_cus)
+{
+    const int64_t most = std::max<int64_t>(1, std::min<int64_t>(VECTOR_DW_PARTS, (16 << 20) / (out_f * in_f * 4)));
+    return (int)std::min<int64_t>(product_room(out_f, in_f, tokens, num_cus), most);
+}
+// scratch: dx's partial matrices and dW's (or dW); 0: not taken
+int64_t vector_products_workspace(int64_t tokens, int64_t in_f, int64_t out_f, bool want_dx)
+{
+    if (!vector_products_ok(tokens, in_f, out_f)) return 0;
+    const int num_cus = num_compute_units(), r = want_dx ? product_room(tokens, in_f, out_f, num_cus) : 1;
+    return (r > 1 ? r : 0) * up256(tokens * in_f * 4) + vector_dw_room(tokens, in_f, out_f, num_cus) * up256(out_f * in_f * 4);
+}
+int vector_products(float *dx, const float *dy, int64_t lddy, const float *x, int64_t ldx, const float *W, int64_t tokens, int64_t in_f, int64_t out_f,
+                    void *workspace, FgSum *dx_sum, VectorDW *dw, hipStream_t s)
+{
+    if (!vector_products_ok(tokens, in_f, out_f) || tokens * lddy >= (1ll << 29) || tokens * ldx >= (1ll << 29)) return RDB_E_UNSUPPORTED;
+    const int num_cus = num_compute_units(), room = dx ? product_room(tokens, in_f, out_f, num_cus) : 1, dw_room = vector_dw_room(tokens, in_f, out_f, num_cus);
+    const int64_t dx_stride = up256(tokens * in_f * 4) / 4, dw_stride = up256(out_f * in_f * 4) / 4;
+    float *dx_part = static_cast<float *>(workspace), *dw_part = dx_part + (room > 1 ? room : 0) * dx_stride;
+    FgProduct qx = {dy, lddy, (tokens - 1) * lddy + out_f, W, in_f, out_f * in_f, dx, in_f, nullptr, tokens, in_f, out_f, 0, 0, 0, 0, 0u};
+    FgProduct qw = {dy, lddy, (tokens - 1) * lddy + out_f, x, ldx, (tokens - 1) * ldx + in_f, dw_part, in_f, nullptr, out_f, in_f, tokens, 0, 0, 0, 0, 0u};
+    *dx_sum = {};
+    auto ranges = [](FgProduct &q, int r, float *part, int64_t stride) {
+        q.kchunk = r > 1 ? fg_chunk(q.K, r) : 0;
+        if (r > 1) {
+            q.out = part;
+            q.split_stride = stride;
+        }
+    };
+    if (dx) {
+        const FgPairPlan plan = fg_plan_pair({qx.M, qw.M}, {qx.N, qw.N}, {qx.K, qw.K}, num_cus, {room, dw_room}, false);
+        FgProduct tx = qx, tw = qw;
+        tx.bm = tw.bm = plan.bm;
+        tx.groups = tw.groups = plan.groups;
+        ranges(tx, plan.ranges[0], dx_part, dx_stride);
+        ranges(tw, plan.ranges[1], dw_part, dw_stride);
+        const int rc = fg_launch_pair(tx, tw, s);
+        if (rc != RDB_E_UNSUPPORTED) {
+            *dx_sum = fg_sum(dx, 0, dx_part, qx.M * qx.N, dx_stride, plan.ranges[0]);
+            *dw = {dw_part, dw_stride, plan.ranges[1]};
+            return rc;
+        }
+        const FgPlan px = fg_plan(qx.M, qx.N, qx.K, num_cus, room, FgGroups<FG_KCONT, FG_MCONT>::four);
+        qx.bm = px.bm;
+        qx.groups = px.groups;
+        ranges(qx, px.ranges, dx_part, dx_stride);
+        if (int rx = fg_launch<FG_KCONT, FG_MCONT>(qx, num_cus, s, "f32_gemm_kernel (dx = dy . W)")) return rx;
+        *dx_sum = fg_sum(dx, 0, dx_part, qx.M * qx.N, dx_stride, px.ranges);
+    }
+    const FgPlan pw = fg_plan(qw.M, qw.N, qw.K, num_cus, dw_room, FgGroups<FG_MCONT, FG_MCONT>::four);
+    qw.bm = pw.bm;
+    qw.groups = pw.groups;
+    ranges(qw, pw.ranges, dw_part, dw_stride);
+    *dw = {dw_part, dw_stride, pw.ranges};
+    return fg_launch<FG_MCONT, FG_MCONT>(qw, num_cus, s, "f32_gemm_kernel (dW = dy^T . x)");
+}
 
 }  // namespace rdb
 

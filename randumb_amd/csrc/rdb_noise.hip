@@ -1,6 +1,7 @@
 // Noise probes, materialise forward/backward, random-bias gradient and embedding gather for gfx950.
 // These are the HBM-facing ops of the pseudorandom tensor (the fused linear kernels live in rdb_linear.hip).
 #include "rdb_common.hpp"
+#include "rdb_sums.hpp"
 #include <algorithm>
 #include <type_traits>
 
@@ -62,7 +63,6 @@ constexpr int COEF_CHUNK = 2048;
 constexpr float MAT_LARGE = 3.777893186295716e22f;   // 2^75
 constexpr int MAT_UNROLL = 16;
 constexpr int MAT_SHORT = 48;
-constexpr int64_t MAT_PAIR_HASHES = (int64_t)1 << 27;   // a weight and its bias in one launch: up to some 45 us of hashing
 
 struct MatVecParams {
     float *out;
@@ -162,8 +162,13 @@ template <int LANES, bool SHORT> __global__ __launch_bounds__(NT) void materiali
 {
     __shared__ __align__(16) float cs[COEF_CHUNK + MAT_UNROLL];   // reads run a turn ahead
     bool one_factor = false;
-    if (blockIdx.x < bias_blocks) materialize_vec_block<false, 16, false>(bias, cs, blockIdx.x, true, one_factor);
-    else materialize_vec_block<false, LANES, SHORT>(weight, cs, blockIdx.x - bias_blocks, true, one_factor);
+    if (blockIdx.x < bias_blocks) {
+        materialize_vec_block<false, 16, false>(bias, cs, blockIdx.x, true, one_factor);
+        return;
+    }
+    const unsigned first = blockIdx.x - bias_blocks;
+    for (unsigned block = first; block < weight.blocks; block += gridDim.x - bias_blocks)
+        materialize_vec_block<false, LANES, SHORT>(weight, cs, block, block == first || weight.k > COEF_CHUNK, one_factor);
 }
 
 // Matrix-coef materialise, arbitrary view: one thread per output element (no sharing of noise between rows).
@@ -320,6 +325,63 @@ __device__ __forceinline__ double block_sum_ll(long long v, long long *scratch)
     return (double)(scratch[0] + scratch[1] + scratch[2] + scratch[3]);
 }
 
+// ----------------------------------------------------------------------------------------------- column sums
+constexpr int BIAS_M = 4, BIAS_MAX_CHUNKS = 16;
+__device__ __forceinline__ float to_f32(float v) { return v; }
+__device__ __forceinline__ float to_f32(bf16_t v) { return bf16_to_f32(v); }
+static int bias_chunks(int64_t rows) { return (int)std::min<int64_t>(BIAS_MAX_CHUNKS, std::max<int64_t>(1, cdiv(rows, 32))); }
+
+// block (bx, by): 64 V columns of a chunk of rows; sh: 256 V floats
+template <typename T, int V>
+__device__ __forceinline__ void column_sums_block(float *__restrict__ part, const T *__restrict__ dy, int64_t ldy, int64_t rows, int64_t n, int64_t per_chunk, int bx, int by,
+                                                  float (*sh)[64 * V])
+{
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t c = ((int64_t)bx * 64 + lane) * V, r0 = (int64_t)by * per_chunk, r1 = r0 + per_chunk < rows ? r0 + per_chunk : rows;
+    float sum[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) sum[j] = 0.0f;
+    if (c < n) {
+        constexpr int AHEAD = 8;   // rows in flight
+        for (int64_t r = r0 + wave; r < r1; r += 4 * AHEAD) {
+            float v[AHEAD][V];
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) {
+                const int64_t row = r + 4 * i;
+                const bool in = row < r1;
+                const T *src = dy + (in ? row : r) * ldy + c;
+                if constexpr (V == 1) {
+                    v[i][0] = to_f32(src[0]);
+                } else {
+                    T raw[V];
+                    __builtin_memcpy(raw, __builtin_assume_aligned(src, 16), sizeof raw);
+#pragma unroll
+                    for (int j = 0; j < V; ++j) v[i][j] = to_f32(raw[j]);
+                }
+#pragma unroll
+                for (int j = 0; j < V; ++j) v[i][j] = in ? v[i][j] : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i)
+#pragma unroll
+                for (int j = 0; j < V; ++j) sum[j] += v[i][j];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < V; ++j) sh[wave][lane * V + j] = sum[j];
+    __syncthreads();
+    for (int i = threadIdx.x; i < 64 * V; i += NT) {
+        const int64_t o = (int64_t)bx * 64 * V + i;
+        if (o < n) part[(int64_t)by * n + o] = (sh[0][i] + sh[1][i]) + (sh[2][i] + sh[3][i]);
+    }
+}
+template <typename T, int V> __global__ __launch_bounds__(NT) void column_sums_kernel(float *__restrict__ part, const T *__restrict__ dy, int64_t ldy, int64_t rows, int64_t n,
+                                                                                    int64_t per_chunk)
+{
+    __shared__ float sh[4][64 * V];
+    column_sums_block<T, V>(part, dy, ldy, rows, n, per_chunk, blockIdx.x, blockIdx.y, sh);
+}
+
 // Vector-coef coefficient gradient / embedding gradient.
 //   dcoef[m] = sum_e noise(PRIME*a(e) + m) * d[e],  a(e) = e  or  idx[e / Q]*Q + e % Q.
 // A block owns a span of elements, whose digits go through LDS 256 at a time (their scale found in a pass of its own over the span),
@@ -334,6 +396,15 @@ struct GradVecParams {
     int64_t k, Nw, span, Q;
     int d_dtype, narrow;
     uint32_t seed;
+    // LAYER: d is the sum of `parts` matrices, fp32, part_stride floats apart; the grid is one-dimensional, mblocks along the coefficients, and behind
+    // the gradient's blocks come those that add up dx, and those of the column sums of dy (col_x along its columns)
+    int parts, mblocks, main_blocks;
+    int64_t part_stride;
+    FgSum sum;
+    float *col_part;
+    const float *dy;
+    int64_t lddy, rows, n, per_chunk;
+    int col_x, col_vec;
 };
 
 template <bool GATHER> __device__ __forceinline__ uint32_t gradvec_offset(const GradVecParams &p, int64_t e)
@@ -343,7 +414,7 @@ template <bool GATHER> __device__ __forceinline__ uint32_t gradvec_offset(const 
     return (uint32_t)(p.idx[j] * p.Q + (e - j * p.Q));
 }
 
-template <bool GATHER, int MT, int WM> __global__ __launch_bounds__(NT) void coef_grad_vec_kernel(GradVecParams p)
+template <bool GATHER, int MT, int WM, bool LAYER> __global__ __launch_bounds__(NT) void coef_grad_vec_kernel(GradVecParams p)
 {
     constexpr int WE = 4 / WM, MBLOCK = 16 * MT * WM, LD = NT + 8;   // LD: 16 bytes of padding, so that 16 rows' pieces lie in different banks
     __shared__ __align__(16) unsigned short win[16][LD];   // rows 0 .. 7: the windows' lower halves, 8 .. 15: their upper halves
@@ -351,19 +422,56 @@ template <bool GATHER, int MT, int WM> __global__ __launch_bounds__(NT) void coe
     __shared__ uint32_t tops[4];
     __shared__ long long sums[4];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, grp = lane >> 4;
-    const int64_t e_begin = (int64_t)blockIdx.y * p.span, e_end = (e_begin + p.span < p.Nw) ? e_begin + p.span : p.Nw;
-    const int64_t m_block = (int64_t)blockIdx.x * MBLOCK, m0 = m_block + (wave % WM) * (16 * MT) + (lane & 15);
-    float *row = p.partial + ((int64_t)blockIdx.y * WE + wave / WM) * p.k;
+    int bx = blockIdx.x, by = blockIdx.y;
+    if constexpr (LAYER) {
+        const int b = blockIdx.x;
+        if (b >= p.main_blocks + p.sum.blocks) {
+            const int c = b - p.main_blocks - p.sum.blocks, cy = c / p.col_x, cx = c - cy * p.col_x;
+            if (p.col_vec) column_sums_block<float, 4>(p.col_part, p.dy, p.lddy, p.rows, p.n, p.per_chunk, cx, cy, reinterpret_cast<float (*)[256]>(win));
+            else column_sums_block<float, 1>(p.col_part, p.dy, p.lddy, p.rows, p.n, p.per_chunk, cx, cy, reinterpret_cast<float (*)[64]>(win));
+            return;
+        }
+        if (b >= p.main_blocks) {
+            f32_sum_block(p.sum, b - p.main_blocks);
+            return;
+        }
+        by = b / p.mblocks;
+        bx = b - by * p.mblocks;
+    }
+    constexpr int RAW = LAYER ? VECTOR_DW_PARTS : 1;
+    auto raw_d = [&](int64_t e, float (&v)[RAW]) {
+        if constexpr (LAYER) {
+#pragma unroll
+            for (int r = 0; r < RAW; ++r) v[r] = r < p.parts ? static_cast<const float *>(p.d)[r * p.part_stride + e] : 0.0f;   // uniform
+        } else {
+            v[0] = load_as_f32(p.d, p.d_dtype, e);
+        }
+    };
+    auto sum_d = [&](const float (&v)[RAW]) {   // in range order
+        float s = v[0];
+#pragma unroll
+        for (int r = 1; r < RAW; ++r)
+            if (r < p.parts) s += v[r];
+        return s;
+    };
+    auto load_d = [&](int64_t e) {
+        float v[RAW];
+        raw_d(e, v);
+        return sum_d(v);
+    };
+    const int64_t e_begin = (int64_t)by * p.span, e_end = (e_begin + p.span < p.Nw) ? e_begin + p.span : p.Nw;
+    const int64_t m_block = (int64_t)bx * MBLOCK, m0 = m_block + (wave % WM) * (16 * MT) + (lane & 15);
+    float *row = p.partial + ((int64_t)by * WE + wave / WM) * p.k;
     uint32_t top = 0;
-    for (int64_t e = e_begin + t; e < e_end; e += NT) top = max(top, __float_as_uint(load_as_f32(p.d, p.d_dtype, e)) & 0x7fffffffu);
+    for (int64_t e = e_begin + t; e < e_end; e += NT) top = max(top, __float_as_uint(load_d(e)) & 0x7fffffffu);
     top = block_max_bits(top, tops);
     if (top >= 0x7f800000u) {   // infinities or NaNs, which have to come out where they belong: a term at a time in fp32
         const int64_t m_end = m_block + MBLOCK < p.k ? m_block + MBLOCK : p.k;
         for (int64_t m = m_block + t; m < m_end; m += NT) {
             float acc = 0.0f;
             for (int64_t e = e_begin; e < e_end; ++e)
-                acc = fmaf(noise2d(gradvec_offset<GATHER>(p, e), (uint32_t)m, p.seed), load_as_f32(p.d, p.d_dtype, e), acc);
-            for (int r = 0; r < WE; ++r) p.partial[((int64_t)blockIdx.y * WE + r) * p.k + m] = r ? 0.0f : acc;
+                acc = fmaf(noise2d(gradvec_offset<GATHER>(p, e), (uint32_t)m, p.seed), load_d(e), acc);
+            for (int r = 0; r < WE; ++r) p.partial[((int64_t)by * WE + r) * p.k + m] = r ? 0.0f : acc;
         }
         return;
     }
@@ -380,20 +488,21 @@ template <bool GATHER, int MT, int WM> __global__ __launch_bounds__(NT) void coe
     uint32_t mask = Q_MASK;
     asm("" : "+v"(mask));   // stays in a vector register
     const int pairs = lane & 8 ? (int)0xeeeeeeeeu : 0x44444444;   // which two of an element's bytes this lane's row has: 2 and 3, or 0 and 1
-    float next_d;
+    float next_d[RAW];
     uint32_t next_a;
     auto fetch = [&](int64_t e0) {
         const int64_t e = e0 + t;
-        next_d = 0.0f;   // zero beyond the span, so the tail adds nothing
+#pragma unroll
+        for (int r = 0; r < RAW; ++r) next_d[r] = 0.0f;   // zero beyond the span, so the tail adds nothing
         next_a = 0;
         if (e < e_end) {
-            next_d = load_as_f32(p.d, p.d_dtype, e);
+            raw_d(e, next_d);
             next_a = gradvec_offset<GATHER>(p, e);
         }
     };
     fetch(e_begin);
     for (int64_t e0 = e_begin; e0 < e_end; e0 += NT) {
-        const float dv = next_d;
+        const float dv = sum_d(next_d);
         const uint32_t a = next_a;
         fetch(e0 + NT);   // while this one is hashed
         uint32_t w[8];
@@ -450,12 +559,11 @@ template <bool GATHER, int MT, int WM> __global__ __launch_bounds__(NT) void coe
 
 // out[c] = sum_r partial[r*cols + c] in a fixed order: 32 columns a block, 32 threads a column that take every 32nd row each (the
 // rows of a gradient's thousand blocks: one thread a column took 60 us), their sums added in thread order.
-__global__ __launch_bounds__(1024) void reduce_rows_kernel(float *__restrict__ out, const float *__restrict__ partial,
-                                                           int64_t rows, int64_t cols)
+__device__ __forceinline__ void reduce_rows_block(float *__restrict__ out, const float *__restrict__ partial, int64_t rows, int64_t cols, int block)
 {
     __shared__ float part[32][33];
     const int cl = threadIdx.x & 31, rg = threadIdx.x >> 5;
-    const int64_t c = (int64_t)blockIdx.x * 32 + cl;
+    const int64_t c = (int64_t)block * 32 + cl;
     float s = 0.0f;
     if (c < cols) {
 #pragma unroll 8
@@ -467,6 +575,10 @@ __global__ __launch_bounds__(1024) void reduce_rows_kernel(float *__restrict__ o
 #pragma unroll
     for (int j = 1; j < 32; ++j) s += part[j][cl];
     out[c] = s;
+}
+__global__ __launch_bounds__(1024) void reduce_rows_kernel(float *__restrict__ out, const float *__restrict__ partial, int64_t rows, int64_t cols)
+{
+    reduce_rows_block(out, partial, rows, cols, blockIdx.x);
 }
 
 // Matrix-coef coefficient gradient: dC[o, m] = sum_i noise(i, m) * dW[o, i].
@@ -586,14 +698,14 @@ static int launch_materialize_vec(float *out, const void *coef, int coef_dtype, 
     return check_launch("materialize_vec_kernel");
 }
 
-template <bool GATHER> static void launch_grad_vec(const GradVecParams &p, dim3 grid, hipStream_t s)
+template <bool GATHER, bool LAYER = false> static void launch_grad_vec(const GradVecParams &p, dim3 grid, hipStream_t s)
 {
     switch (grad_block(p.k)) {
-    case 16: coef_grad_vec_kernel<GATHER, 1, 1><<<grid, NT, 0, s>>>(p); break;
-    case 32: coef_grad_vec_kernel<GATHER, 1, 2><<<grid, NT, 0, s>>>(p); break;
-    case 64: coef_grad_vec_kernel<GATHER, 1, 4><<<grid, NT, 0, s>>>(p); break;
-    case 128: coef_grad_vec_kernel<GATHER, 2, 4><<<grid, NT, 0, s>>>(p); break;
-    default: coef_grad_vec_kernel<GATHER, 4, 4><<<grid, NT, 0, s>>>(p); break;
+    case 16: coef_grad_vec_kernel<GATHER, 1, 1, LAYER><<<grid, NT, 0, s>>>(p); break;
+    case 32: coef_grad_vec_kernel<GATHER, 1, 2, LAYER><<<grid, NT, 0, s>>>(p); break;
+    case 64: coef_grad_vec_kernel<GATHER, 1, 4, LAYER><<<grid, NT, 0, s>>>(p); break;
+    case 128: coef_grad_vec_kernel<GATHER, 2, 4, LAYER><<<grid, NT, 0, s>>>(p); break;
+    default: coef_grad_vec_kernel<GATHER, 4, 4, LAYER><<<grid, NT, 0, s>>>(p); break;
     }
 }
 static int launch_reduce_rows(float *out, const float *partial, int64_t rows, int64_t cols, hipStream_t s)
@@ -680,14 +792,14 @@ extern "C" int rdb_materialize_weight_and_bias(float *weight, int64_t n, const f
         return set_error(RDB_E_SHAPE, "%s: n=%lld k=%lld, bias n=%lld k=%lld", who, (long long)n, (long long)k, (long long)bias_n, (long long)bias->k);
     if ((n > 0 && (!weight || (!coef && k > 0))) || (bias_n > 0 && (!bias->values || (!bias->coef && bias->k > 0)))) return set_error(RDB_E_NULL, "%s: an output or its coefficients are NULL", who);
     hipStream_t s = (hipStream_t)stream;
-    // Side by side where both are short; a long one's kernel stays as it is, and so do biases that get another number of lanes.
-    if (n > 0 && bias_n > 0 && n * std::max<int64_t>(k, 1) <= MAT_PAIR_HASHES && mat_lanes(bias_n, bias->k) == 16) {
+    // side by side, but for biases that get another number of lanes
+    if (n > 0 && bias_n > 0 && mat_lanes(bias_n, bias->k) == 16) {
         const auto params = [](float *out, const float *c, const float *sc, int64_t terms, int64_t len, uint32_t sd) {
-            return MatVecParams{out, c, sc, nullptr, terms, len, len, 0, 1, RDB_F32, len < (1ll << 32), 1, sd, 0};
+            return MatVecParams{out, c, sc, nullptr, terms, len, len, 0, 1, RDB_F32, len < (1ll << 32), 1, sd, (unsigned)cdiv(len * mat_lanes(len, terms), NT)};
         };
         const MatVecParams w = params(weight, coef, scale, k, n, seed), b = params(bias->values, bias->coef, bias->scale, bias->k, bias_n, bias->seed);
         const int lanes = mat_lanes(n, k);
-        const unsigned bias_blocks = (unsigned)cdiv(bias_n * 16, NT), blocks = bias_blocks + (unsigned)cdiv(n * lanes, NT);
+        const unsigned bias_blocks = b.blocks, blocks = bias_blocks + std::min(w.blocks, 8u * (unsigned)num_compute_units());
         auto launch = [&](auto lanes_) {
             constexpr int L = decltype(lanes_)::value;
             if (k <= MAT_SHORT) materialize_vec_pair_kernel<L, true><<<blocks, NT, 0, s>>>(w, b, bias_blocks);
@@ -725,7 +837,8 @@ static int coef_grad_vec(float *dcoef, const void *d, int d_dtype, int64_t k, in
         partial = (float *)workspace;
     }
     const dim3 grid((unsigned)cdiv(k, grad_block(k)), (unsigned)(splits / grad_rows(k)));
-    const GradVecParams p = {partial, d, idx, k, Nw, span, Q, d_dtype, Nw < (1ll << 32) && Q < (1ll << 32), seed};
+    GradVecParams p = {partial, d, idx, k, Nw, span, Q, d_dtype, Nw < (1ll << 32) && Q < (1ll << 32), seed};
+    p.parts = 1;
     if (idx) launch_grad_vec<true>(p, grid, s);
     else launch_grad_vec<false>(p, grid, s);
     int rc = check_launch("coef_grad_vec_kernel");
@@ -853,55 +966,6 @@ extern "C" int rdb_embed_bwd(float *dcoef, const int64_t *idx, int64_t n_idx, co
 // 6.0 us; 1024 tokens x 3072, k = 256: 19 -> 12 us.
 namespace rdb {
 
-constexpr int BIAS_M = 4, BIAS_MAX_CHUNKS = 16;
-__device__ __forceinline__ float to_f32(float v) { return v; }
-__device__ __forceinline__ float to_f32(bf16_t v) { return bf16_to_f32(v); }
-static int bias_chunks(int64_t rows) { return (int)std::min<int64_t>(BIAS_MAX_CHUNKS, std::max<int64_t>(1, cdiv(rows, 32))); }
-
-template <typename T, int V> __global__ __launch_bounds__(NT) void column_sums_kernel(float *__restrict__ part, const T *__restrict__ dy, int64_t ldy, int64_t rows, int64_t n,
-                                                                                    int64_t per_chunk)
-{
-    __shared__ float sh[4][64 * V];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int64_t c = ((int64_t)blockIdx.x * 64 + lane) * V, r0 = (int64_t)blockIdx.y * per_chunk, r1 = r0 + per_chunk < rows ? r0 + per_chunk : rows;
-    float sum[V];
-#pragma unroll
-    for (int j = 0; j < V; ++j) sum[j] = 0.0f;
-    if (c < n) {
-        constexpr int AHEAD = 8;   // rows in flight
-        for (int64_t r = r0 + wave; r < r1; r += 4 * AHEAD) {
-            float v[AHEAD][V];
-#pragma unroll
-            for (int i = 0; i < AHEAD; ++i) {
-                const int64_t row = r + 4 * i;
-                const bool in = row < r1;
-                const T *src = dy + (in ? row : r) * ldy + c;
-                if constexpr (V == 1) {
-                    v[i][0] = to_f32(src[0]);
-                } else {
-                    T raw[V];
-                    __builtin_memcpy(raw, __builtin_assume_aligned(src, 16), sizeof raw);
-#pragma unroll
-                    for (int j = 0; j < V; ++j) v[i][j] = to_f32(raw[j]);
-                }
-#pragma unroll
-                for (int j = 0; j < V; ++j) v[i][j] = in ? v[i][j] : 0.0f;
-            }
-#pragma unroll
-            for (int i = 0; i < AHEAD; ++i)
-#pragma unroll
-                for (int j = 0; j < V; ++j) sum[j] += v[i][j];
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < V; ++j) sh[wave][lane * V + j] = sum[j];
-    __syncthreads();
-    for (int i = threadIdx.x; i < 64 * V; i += NT) {
-        const int64_t o = (int64_t)blockIdx.x * 64 * V + i;
-        if (o < n) part[(int64_t)blockIdx.y * n + o] = (sh[0][i] + sh[1][i]) + (sh[2][i] + sh[3][i]);
-    }
-}
-
 // What a block of the gradient does with a column's sum g (block b: coefficients b * BIAS_M .. + 3; the block behind the last
 // coefficient: the scale), and at the end with its threads' shares.
 __device__ __forceinline__ void bias_contract(float (&acc)[BIAS_M], float g, uint32_t o, int64_t m0, bool scale, uint32_t seed)
@@ -973,10 +1037,11 @@ template <typename T> __global__ __launch_bounds__(1024) void bias_grad_direct_k
 
 // The second launch.  THREADS: a thread's outputs are a chain of
 // memory latencies, so long biases take blocks of 1024 (3072 outputs, k = 256: 15.7 us with 256 threads, 12 turns of the loop; vector-coef layer step 561 -> 540).
-template <int THREADS> __global__ __launch_bounds__(THREADS) void bias_grad_kernel(float *__restrict__ dcoef, float *__restrict__ ds, const float *__restrict__ part, int chunks, int64_t n, int64_t k,
-                                                       uint32_t seed)
+template <int THREADS>
+__device__ __forceinline__ void bias_grad_block(float *__restrict__ dcoef, float *__restrict__ ds, const float *__restrict__ part, int chunks, int64_t n, int64_t k, uint32_t seed,
+                                                int block)
 {
-    const int64_t m0 = (int64_t)blockIdx.x * BIAS_M;
+    const int64_t m0 = (int64_t)block * BIAS_M;
     const bool scale = !dcoef || m0 >= k;
     float acc[BIAS_M] = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int64_t o = threadIdx.x; o < n; o += THREADS) {
@@ -991,6 +1056,18 @@ template <int THREADS> __global__ __launch_bounds__(THREADS) void bias_grad_kern
         bias_contract(acc, g, (uint32_t)o, m0, scale, seed);
     }
     bias_finish<THREADS>(acc, dcoef, ds, m0, k, scale);
+}
+template <int THREADS> __global__ __launch_bounds__(THREADS) void bias_grad_kernel(float *__restrict__ dcoef, float *__restrict__ ds, const float *__restrict__ part, int chunks, int64_t n, int64_t k,
+                                                       uint32_t seed)
+{
+    bias_grad_block<THREADS>(dcoef, ds, part, chunks, n, k, seed, blockIdx.x);
+}
+// The end of a vector-coef layer's backward pass: the partial rows of its coefficients' gradient, and behind them its bias's blocks
+__global__ __launch_bounds__(1024) void layer_grads_kernel(float *__restrict__ dcoef, const float *__restrict__ partial, int64_t rows, int64_t k, int row_blocks,
+                                                           float *__restrict__ db, const float *__restrict__ part, int chunks, int64_t n, int64_t bias_k, uint32_t bias_seed)
+{
+    if ((int)blockIdx.x < row_blocks) reduce_rows_block(dcoef, partial, rows, k, blockIdx.x);
+    else bias_grad_block<1024>(db, nullptr, part, chunks, n, bias_k, bias_seed, (int)blockIdx.x - row_blocks);
 }
 
 }  // namespace rdb
@@ -1037,4 +1114,94 @@ extern "C" int rdb_bias_bwd(float *dcoef, float *ds, const void *dy, int dtype, 
     if (n > 512) bias_grad_kernel<1024><<<(unsigned)blocks, 1024, 0, s>>>(dcoef, ds, part, chunks, n, k, seed);
     else bias_grad_kernel<NT><<<(unsigned)blocks, NT, 0, s>>>(dcoef, ds, part, chunks, n, k, seed);
     return check_launch("bias_grad_kernel");
+}
+
+// ----------------------------------------------------------------------------------------------- backward pass of a vector-coef layer
+// As calls of their own: dx and dW, a product and a sum of its ranges each, dW's contraction with the noise and the sum of its partial rows, the
+// column sums of dy and the bias's contraction, eight launches of which six are 5 to 8 us and a gap behind each.  Here four: the two products side by
+// side, the contraction, which adds dW's ranges up on the way and has dx's sums and the column sums beside it (it is the vector ALU's, they are the memory's), and the
+// small ends together.  Step of 1024 tokens x 768 -> 3072, k = 256: 481 -> 466 us (1.3 % of it for the bias's values formed beside W's in the forward pass); 1024 x 512 ->
+// 1024, k = 200: 131 -> 118; steps that wait for the host, 2048 x 256 -> 512, k = 100: 100 -> 81; 32 x 64 -> 64, k = 16: 90 -> 79.
+namespace rdb {
+
+struct VectorBwdPlan {
+    int64_t products, rows_at, cols_at, bytes, splits, span;
+    int chunks;
+};
+static bool vector_bwd_plan(VectorBwdPlan &v, int64_t tokens, int64_t in_f, int64_t out_f, int64_t k, bool want_dx, bool bias)
+{
+    if (tokens <= 0 || in_f <= 0 || out_f <= 0 || k <= 0 || out_f * in_f >= (1ll << 31)) return false;
+    v.products = vector_products_workspace(tokens, in_f, out_f, want_dx);
+    if (!v.products) return false;
+    split_plan(out_f * in_f, k, &v.splits, &v.span);
+    auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
+    v.rows_at = v.products;
+    v.cols_at = v.rows_at + (v.splits > 1 ? up(v.splits * k * 4) : 0);
+    v.chunks = bias_chunks(tokens);
+    v.bytes = v.cols_at + (bias ? up((int64_t)v.chunks * out_f * 4) : 0);
+    return true;
+}
+
+}  // namespace rdb
+
+extern "C" int64_t rdb_vector_linear_bwd_workspace_bytes(int64_t tokens, int64_t in_f, int64_t out_f, int64_t k, int want_dx, int want_bias)
+{
+    VectorBwdPlan v;
+    return vector_bwd_plan(v, tokens, in_f, out_f, k, want_dx != 0, want_bias != 0) ? v.bytes : 0;
+}
+
+extern "C" int rdb_vector_linear_bwd(float *dx, float *dcoef, float *dbias_coef, const float *dy, int64_t lddy, const float *x, int64_t ldx, const float *W, int64_t tokens,
+                                     int64_t in_f, int64_t out_f, int64_t k, uint32_t seed, int64_t bias_k, uint32_t bias_seed, void *workspace, int64_t workspace_bytes,
+                                     void *stream)
+{
+    const char *who = "rdb_vector_linear_bwd";
+    if (tokens < 0 || in_f < 0 || out_f < 0 || k < 0 || bias_k < 0 || lddy < out_f || ldx < in_f)
+        return set_error(RDB_E_SHAPE, "%s: tokens=%lld in_f=%lld out_f=%lld k=%lld bias k=%lld lddy=%lld ldx=%lld", who, (long long)tokens, (long long)in_f, (long long)out_f,
+                         (long long)k, (long long)bias_k, (long long)lddy, (long long)ldx);
+    if (!dcoef || !dy || !x || (dx && !W)) return set_error(RDB_E_NULL, "%s: dcoef, dy, x or (with dx) W is NULL", who);
+    VectorBwdPlan v;
+    const bool bias = dbias_coef && bias_k > 0;
+    if (!vector_bwd_plan(v, tokens, in_f, out_f, k, dx != nullptr, bias))
+        return set_error(RDB_E_UNSUPPORTED, "%s: needs non-empty sizes, matrices of less than 2^29 elements and the split products (rdb_set_f32_split)", who);
+    if (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < v.bytes)
+        return set_error(RDB_E_WORKSPACE, "%s: workspace of %lld bytes needed, %lld given", who, (long long)v.bytes, (long long)workspace_bytes);
+    hipStream_t s = (hipStream_t)stream;
+    char *ws = static_cast<char *>(workspace);
+    GradVecParams p = {};
+    VectorDW dw;
+    int rc = vector_products(dx, dy, lddy, x, ldx, W, tokens, in_f, out_f, ws, &p.sum, &dw, s);
+    if (rc == RDB_E_UNSUPPORTED) return set_error(rc, "%s: matrices of less than 2^29 elements", who);
+    if (rc) return rc;
+    float *rows = v.splits > 1 ? reinterpret_cast<float *>(ws + v.rows_at) : dcoef, *cols = reinterpret_cast<float *>(ws + v.cols_at);
+    p.partial = rows;
+    p.d = dw.part;
+    p.parts = dw.parts;
+    p.part_stride = dw.stride;
+    p.k = k;
+    p.Nw = out_f * in_f;
+    p.span = v.span;
+    p.Q = 1;
+    p.d_dtype = RDB_F32;
+    p.narrow = 1;
+    p.seed = seed;
+    p.mblocks = (int)cdiv(k, grad_block(k));
+    p.main_blocks = p.mblocks * (int)(v.splits / grad_rows(k));
+    unsigned blocks = (unsigned)(p.main_blocks + p.sum.blocks);
+    if (bias) {
+        p.col_part = cols;
+        p.dy = dy;
+        p.lddy = lddy;
+        p.rows = tokens;
+        p.n = out_f;
+        p.per_chunk = cdiv(tokens, v.chunks);
+        p.col_vec = ((uintptr_t)dy & 15) == 0 && lddy % 4 == 0 && out_f % 4 == 0;
+        p.col_x = (int)cdiv(out_f, p.col_vec ? 256 : 64);
+        blocks += (unsigned)(p.col_x * v.chunks);
+    }
+    launch_grad_vec<false, true>(p, dim3(blocks), s);
+    if ((rc = check_launch("coef_grad_vec_kernel"))) return rc;
+    const int row_blocks = v.splits > 1 ? (int)cdiv(k, 32) : 0, bias_blocks = bias ? (int)cdiv(bias_k, BIAS_M) : 0;
+    if (!(row_blocks + bias_blocks)) return RDB_OK;
+    layer_grads_kernel<<<(unsigned)(row_blocks + bias_blocks), 1024, 0, s>>>(dcoef, rows, v.splits, k, row_blocks, dbias_coef, cols, v.chunks, out_f, bias_k, bias_seed);
+    return check_launch("layer_grads_kernel");
 }

@@ -733,19 +733,43 @@ class VectorLinear : public Function<VectorLinear> {
             const auto db = bm[0] < 0 ? std::pair<Tensor, Tensor>() : bias_grads_with_graph(dy, bm);
             return {dx, dc, ds, db.first, db.second, Tensor(), Tensor()};
         }
+        const auto bm = ctx->saved_data["bias"].toIntVector();
+        const int bias_at = has_scale ? 3 : 2;
+        Tensor W;
         if (want_x) {
             const bool kept = saved[3].defined();
             if (kept) restored(who, restored_values(who, saved[3], dy, x0.scalar_type(), l.out_f * l.in_f), dy, {l.out_f, l.in_f});
-            const Tensor W = kept ? saved[3] : coef_values(coef, scale, l.out_f * l.in_f, l.seed).view({l.out_f, l.in_f});
-            dx = product(at::empty(x0.sizes(), dy.options()), dy, false, W, true, Tensor());
+            W = kept ? saved[3] : coef_values(coef, scale, l.out_f * l.in_f, l.seed).view({l.out_f, l.in_f});
         }
+        // the gradients that a layer without a fused random bias asks for, together
+        const bool b_coef = bm[0] >= 0 && ctx->needs_input_grad(bias_at), b_scale = bm[0] >= 0 && bm[3] >= 0 && ctx->needs_input_grad(bias_at + 1);
+        if (want_c && !want_s && !b_scale && !(b_coef && bm[1] < 0) && dy.scalar_type() == at::kFloat && x0.scalar_type() == at::kFloat && dy.numel() && x0.numel()) {
+            const int64_t k = coef.numel(), bk = b_coef ? bm[0] : 0, need = rdb_vector_linear_bwd_workspace_bytes(dy.size(0), l.in_f, l.out_f, k, want_x, bk > 0);
+            if (need > 0) {
+                const Tensor x = act(x0.reshape({-1, l.in_f})), ws = bytes(need, dy);
+                const auto f32 = dy.options();
+                if (want_x) dx = at::empty(x0.sizes(), f32);
+                dc = at::empty({k}, f32);
+                Tensor db = b_coef ? at::empty({bk}, f32) : Tensor();
+                const int rc = rdb_vector_linear_bwd(want_x ? dx.data_ptr<float>() : nullptr, dc.data_ptr<float>(), bk > 0 ? db.data_ptr<float>() : nullptr, dy.data_ptr<float>(),
+                                                     dy.stride(0), x.data_ptr<float>(), x.stride(0), want_x ? W.data_ptr<float>() : nullptr, dy.size(0), l.in_f, l.out_f, k,
+                                                     l.seed, bk, (uint32_t)std::max<int64_t>(bm[1], 0), ptr(ws), need, stream_of(dy));
+                if (rc != RDB_E_UNSUPPORTED) {
+                    check(rc, "rdb_vector_linear_bwd");
+                    dc = dc.to(coef.scalar_type());
+                    if (b_coef) db = db.to((at::ScalarType)bm[2]);
+                    return {dx, dc, ds, db, Tensor(), Tensor(), Tensor()};
+                }
+            }
+        }
+        if (want_x) dx = product(at::empty(x0.sizes(), dy.options()), dy, false, W, true, Tensor());
         if (want_c || want_s) {
             const Tensor dW = product(at::empty({l.out_f, l.in_f}, dy.options()), dy, true, act(x0.reshape({-1, l.in_f})), true, Tensor());
             const auto g = coef_grads(dW, coef.numel(), l.seed, want_c, want_s);
             if (want_c) dc = g.first.to(coef.scalar_type());
             if (want_s) ds = g.second.to((at::ScalarType)m[3]);
         }
-        const auto db = bias_grads(ctx, dy, ctx->saved_data["bias"].toIntVector(), has_scale ? 3 : 2);
+        const auto db = bias_grads(ctx, dy, bm, bias_at);
         return {dx, dc, ds, db.first, db.second, Tensor(), Tensor()};
     }
 };

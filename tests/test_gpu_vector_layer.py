@@ -92,3 +92,40 @@ def test_embedding(shape, dim, k):
     dy = torch.randn_like(y)
     got, = torch.autograd.grad(y, [table.weight_coef], dy)
     assert torch.equal(got, ops.embed_bwd(idx, dy, k, dim, 4))
+
+
+@pytest.mark.parametrize("tokens,in_f,out_f,k,bias_k", [(1, 1, 1, 1, 1), (33, 67, 130, 17, 0), (257, 300, 65, 40, 9), (700, 129, 1000, 256, 64), (1500, 300, 520, 100, 300)])
+def test_backward_pass_in_one_call(tokens, in_f, out_f, k, bias_k):
+    """rdb_vector_linear_bwd against fp64 and against the calls it stands for: dx or not, a bias or not, rows that are slices."""
+    from randumb_amd import _lib, hip
+
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(tokens + k)
+    dy = torch.randn(tokens, out_f + 3, generator=g, device="cuda")[:, :out_f]
+    x = torch.randn(tokens, in_f + 1, generator=g, device="cuda")[:, :in_f]
+    W = torch.randn(out_f, in_f, generator=g, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    noise = hip.sq5_fill_2d(out_f * in_f, k, 3).double()
+    want_dc = (dy.double().t() @ x.double()).reshape(-1) @ noise
+    for with_dx in (True, False):
+        need = lib.rdb_vector_linear_bwd_workspace_bytes(tokens, in_f, out_f, k, with_dx, bias_k > 0)
+        assert need > 0
+        ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        dx, dc, db = torch.full((tokens, in_f), 7.0, device="cuda"), torch.empty(k, device="cuda"), torch.empty(max(bias_k, 1), device="cuda")
+
+        def call(bytes_given):
+            return lib.rdb_vector_linear_bwd(dx.data_ptr() if with_dx else None, dc.data_ptr(), db.data_ptr() if bias_k else None, dy.data_ptr(), dy.stride(0), x.data_ptr(),
+                                             x.stride(0), W.data_ptr() if with_dx else None, tokens, in_f, out_f, k, 3, bias_k, 4, ws.data_ptr(), bytes_given, stream)
+
+        assert call(need) == 0
+        first = (dx.clone(), dc.clone(), db.clone())
+        assert call(need) == 0 and all(torch.equal(a, b) for a, b in zip(first[: 2 + (bias_k > 0)], (dx, dc, db)))
+        # sums of products that are exact to 2^-21 or so, dW's rounded to fp32
+        assert _rel(dc, want_dc.cpu()) < 3e-6
+        if with_dx:
+            assert _rel(dx, (dy.double() @ W.double()).cpu()) < 3e-6
+        else:
+            assert bool((dx == 7.0).all())
+        if bias_k:
+            assert _rel(db, (dy.double().sum(0) @ hip.sq5_fill_2d(out_f, bias_k, 4).double()).cpu()) < 3e-6
+        assert call(need - 1) < 0

@@ -28,7 +28,6 @@ int f32_split_mode();   // rdb_f32.hip
 
 constexpr int FEW_ROWS = 64;       // output features of an expanding block: 16 a wave
 constexpr int FEW_COEFS = 16;      // coefficients of a contracting block
-constexpr int FEW_STEPS = 4;       // steps of 32 contraction values a contracting wave hashes ahead of its products
 constexpr int FEW_TOKENS = 256, FEW_K = 512;   // z's three parts of 32 tokens in LDS: at most 100 KB
 
 struct FewParams {
@@ -198,9 +197,10 @@ template <> struct FewSide<float> {
     }
 };
 
-// Block (range, chunk, group): z[TT tiles of tokens][16 coefficients] over the chunk, a quarter of it to a wave.
-template <typename E, int TT> __device__ __forceinline__ void few_contract(const FewParams &p, int b, float *__restrict__ lds)
+// Block (range, chunk, group) of WAVES waves: z[TT tiles of tokens][16 coefficients] over the chunk, each wave its share of it.
+template <typename E, int TT, int WAVES> __device__ __forceinline__ void few_contract(const FewParams &p, int b, float *__restrict__ lds)
 {
+    constexpr int FEW_STEPS = 16 / WAVES;   // steps of 32 contraction values a wave hashes ahead of its products
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
     int range = b % p.ranges, ch = b / p.ranges, group = 0;
     if (TT > 1) {   // a group's chunk is read by blocks of one die where that comes out even
@@ -210,7 +210,7 @@ template <typename E, int TT> __device__ __forceinline__ void few_contract(const
         group = b - range * pieces - ch * p.c_groups;
     }
     const int m = range * FEW_COEFS + r, tile0 = group * TT, t0 = tile0 * 16, T = min(TT * 16, p.T - t0);
-    const int i_begin = (ch * 4 + wave) * p.wave_values;
+    const int i_begin = (ch * WAVES + wave) * p.wave_values;
     const E *const x = static_cast<const E *>(p.x) + (int64_t)t0 * p.ldx;
     const E *row[TT];
     bool live[TT];
@@ -263,20 +263,20 @@ template <typename E, int TT> __device__ __forceinline__ void few_contract(const
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
         const int t = tt * 16 + (tid >> 4);
-        if (t < T) {
+        if (t < T && tid < 256) {
             float *const out = p.part + (((int64_t)ch * p.tiles + tile0 + tt) * p.ranges + range) * p.tile * 16;
             float v = lds[tt * 256 + tid];
 #pragma unroll
-            for (int w = 1; w < 4; ++w) v += lds[(w * TT + tt) * 256 + tid];
+            for (int w = 1; w < WAVES; ++w) v += lds[(w * TT + tt) * 256 + tid];
             __hip_atomic_store(out + tid, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }
 
-// Block: 64 output features, TT tiles of tokens.  MANY: tiles have 16 tokens
-template <typename E, int KS, int TT, bool MANY> __device__ __forceinline__ void few_expand(const FewParams &p, int b, unsigned char *__restrict__ smem)
+// Block: 64 output features, TT tiles of tokens.  MANY: tiles have 16 tokens.  Waves behind the first four (a block as large as a contracting one) add z up and leave
+template <typename E, int KS, int TT, bool MANY, int WAVES> __device__ __forceinline__ void few_expand(const FewParams &p, int b, unsigned char *__restrict__ smem)
 {
-    constexpr int KW = KS * 32, LD = KW + 8;   // 16 bytes of padding: 16 rows' pieces lie in different banks
+    constexpr int THREADS = WAVES * 64, KW = KS * 32, LD = KW + 8;   // 16 bytes of padding: 16 rows' pieces lie in different banks
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
     const int tile = MANY ? 16 : p.tile, tile0 = MANY ? b / p.e_blocks * TT : 0, t0 = tile0 * 16, T = min(TT * 16, p.T - t0), ob = MANY ? b % p.e_blocks : b, o0 = ob * FEW_ROWS + wave * 16;
     bf16_t *const planes = reinterpret_cast<bf16_t *>(smem);
@@ -285,7 +285,7 @@ template <typename E, int KS, int TT, bool MANY> __device__ __forceinline__ void
     // the wave's rows of C, before anything is waited for
     FewRaw<E> c[KS];
     {
-        const bool ok = o0 + r < p.out_f;
+        const bool ok = wave < 4 && o0 + r < p.out_f;
         const E *const row = static_cast<const E *>(p.coef) + (int64_t)(ok ? o0 + r : 0) * p.k;
 #pragma unroll
         for (int s = 0; s < KS; ++s) c[s] = few_load<E>(row, s * 32 + g * 8, p.k, ok, p.c_vec);
@@ -315,7 +315,7 @@ template <typename E, int KS, int TT, bool MANY> __device__ __forceinline__ void
         }
         __syncthreads();
         if (verdict == 0) {   // gave up: the block's share of the output becomes NaN, never a sum of whatever is in memory
-            for (int i = tid; i < T * FEW_ROWS; i += 256) {
+            for (int i = tid; i < T * FEW_ROWS; i += THREADS) {
                 const int t = i / FEW_ROWS, o = ob * FEW_ROWS + i % FEW_ROWS;
                 if (o < p.out_f) elem<E>::store(y + (int64_t)t * p.ldy + o, __uint_as_float(0x7fc00000u));
             }
@@ -329,7 +329,7 @@ template <typename E, int KS, int TT, bool MANY> __device__ __forceinline__ void
     // IB entries of CB chunks in flight
     auto add_up = [&](auto ib_, auto cb_) __attribute__((always_inline)) {
         constexpr int IB = decltype(ib_)::value, CB = decltype(cb_)::value;
-        for (int i0 = tid; i0 < n4; i0 += 256 * IB) {
+        for (int i0 = tid; i0 < n4; i0 += THREADS * IB) {
             f32x4 v[IB];
             for (int c0 = 0; c0 < p.chunks; c0 += CB) {
                 f32x4 u[IB][CB];
@@ -337,7 +337,7 @@ template <typename E, int KS, int TT, bool MANY> __device__ __forceinline__ void
                 for (int i = 0; i < IB; ++i)
 #pragma unroll
                     for (int q = 0; q < CB; ++q) {
-                        const int at = (int)(((int64_t)min(c0 + q, p.chunks - 1) * stride + first + (int64_t)min(i0 + i * 256, n4 - 1) * 4) * 4);
+                        const int at = (int)(((int64_t)min(c0 + q, p.chunks - 1) * stride + first + (int64_t)min(i0 + i * THREADS, n4 - 1) * 4) * 4);
                         u[i][q] = __builtin_bit_cast(f32x4, p.slots ? __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, SCOPE_DEVICE) : __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
                     }
 #pragma unroll
@@ -350,7 +350,7 @@ template <typename E, int KS, int TT, bool MANY> __device__ __forceinline__ void
             }
 #pragma unroll
             for (int i = 0; i < IB; ++i) {
-                const int e = i0 + i * 256;
+                const int e = i0 + i * THREADS;
                 if (e >= n4) continue;
                 const int sub = TT > 1 && (e >> 2) >= per ? 1 : 0, rt = (e >> 2) - sub * per, range = rt / tile, t = sub * 16 + rt - range * tile, m = range * FEW_COEFS + (e & 3) * 4;
 #pragma unroll
@@ -372,11 +372,12 @@ template <typename E, int KS, int TT, bool MANY> __device__ __forceinline__ void
     // coefficients beyond the last range meet zeros of C: they must be finite
     const int tail4 = (KW - p.ranges * FEW_COEFS) / 4;
     if (tail4 > 0)
-        for (int e = tid; e < 3 * T * tail4; e += 256) {
+        for (int e = tid; e < 3 * T * tail4; e += THREADS) {
             const int row = e / tail4, pl = row / T;
             *reinterpret_cast<uint2 *>(planes + pl * PLANE + (row - pl * T) * LD + p.ranges * FEW_COEFS + (e - row * tail4) * 4) = make_uint2(0u, 0u);
         }
     __syncthreads();
+    if (wave >= 4) return;
     f32x4 acc[TT], low[TT];
     auto product = [&](auto any) __attribute__((always_inline)) {
         constexpr bool ANY = decltype(any)::value;
@@ -460,24 +461,36 @@ __global__ __launch_bounds__(256) void few_sum_kernel(float *__restrict__ part, 
 }
 
 // TC, TE: tiles of tokens of a contracting and of an expanding block
-template <typename E, int KS, int TC, int TE> __global__ __launch_bounds__(256, 1) void few_fwd_kernel(FewParams p)
+template <typename E, int KS, int TC, int TE, int WAVES> __global__ __launch_bounds__(WAVES * 64, 1) void few_fwd_kernel(FewParams p)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const int b = blockIdx.x;
     if (b >= p.c_blocks) {
-        few_expand<E, KS, TE, TC == 2>(p, b - p.c_blocks, smem);
+        few_expand<E, KS, TE, TC == 2, WAVES>(p, b - p.c_blocks, smem);
         return;
     }
     if (p.slots && threadIdx.x == 0) __hip_atomic_store(p.slots + b, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // a replay may find its tag
-    few_contract<E, TC>(p, b, reinterpret_cast<float *>(smem));
+    few_contract<E, TC, WAVES>(p, b, reinterpret_cast<float *>(smem));
     if (!p.slots) return;
     if (b == 0 && threadIdx.x == 0) __hip_atomic_store(p.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     publish_tag(p.slots + b, p.tag);
 }
 
+// the contracting blocks of the form in two launches
+template <typename E, int TC, int WAVES> __global__ __launch_bounds__(WAVES * 64, 1) void few_contract_kernel(FewParams p)
+{
+    __shared__ __align__(16) float lds[WAVES * TC * 256];
+    few_contract<E, TC, WAVES>(p, blockIdx.x, lds);
+}
+
 // ----------------------------------------------------------------------------------------------- host side
 // Chunks: about eight of them (sixteen where there is one range of coefficients), of 128 to 512 values (a contracting block hashes a chunk for 16 coefficients: 128 values cost it 0.6 us;
 // an expanding block reads eight at a time: 1 x 4096 -> 4096, k = 16: chunks of 128, 256, 512, 1024: 8.9, 8.0, 8.2, 10.9 us).
+// waves: a wave hashes 32 contraction values for its 16 coefficients, which a SIMD with a single wave does at half its rate, and the blocks are fewer than the chip holds; so
+// a chunk of 512 is 16 waves, or 8 where an expanding block is as large (more have no registers for that; k > 256: four).  us per call, four waves -> so: 16 x 4096 -> 11008, k = 256,
+// bf16 11.4 -> 11.0; 64 tokens 18.6 -> 17.3; 8 x 8192 -> 8192, k = 512 21.9 -> 19.9; in one launch: 1 x 4096 -> 4096, k = 16, fp32 8.9 -> 8.1; 4 x 2000 -> 5000, k = 100 9.5 -> 8.7;
+// 16 x 4096 -> 4096, k = 128 11.1 -> 10.6.  (Chunks of 1024 and 2048 in 16 waves, half and a quarter of the partial sums: 11.8 and 15.1 for the first.  Expanding blocks of eight waves in
+// a launch of their own: 64 tokens 20.7.)  The number depends on the layer alone, so that the same sums come out in one launch and in two.
 // te: tiles of an expanding block.  Finer is sooner ready while the blocks run side by side, two (of k > 128: one) to a compute unit: 64 x
 // 768 -> 3072, k = 64: 8.2 us, two tiles 9.1; 80 x 8192 -> 8192, k = 64, 640 blocks of one tile: 18.7, two tiles 15.1.
 // sum: beyond 200 KB of partial sums for a block they are added up once, by a launch of its own, and not by every expanding block
@@ -485,12 +498,13 @@ template <typename E, int KS, int TC, int TE> __global__ __launch_bounds__(256, 
 // one: a single launch where the expanding blocks are few and the partial sums of each small; tags and reads that go around L2 cost many
 // blocks more than a launch does (16 x 4096 -> 11008, k = 256: two launches 11.5, one 13.5), but a program's host takes 9.0 to 11.7 us (by
 // the box and by what the program does between calls) to issue two, and those calls then take that.  us of a call in one launch, which
-// the host does not hold up: 5 x 1001 -> 999, k = 99: 7.8; 48 x 768 -> 768, k = 64: 8.3; 100 x 264 -> 352, k = 64: 8.7; 32 x 1024 -> 2048,
+// the host does not hold up: (two launches wait for the host, 10.0 and more) 1 x 2048 -> 11008, k = 64, 172 blocks, 32 tags: 8.7; 8 tokens, 16 KB a block: 9.1, but 1 x 4096 ->
+// 11008, k = 256, 128 tags 10.4, 2 x 4096 -> 16000, k = 128, 250 blocks 10.5; earlier, with four waves: 5 x 1001 -> 999, k = 99: 7.8; 48 x 768 -> 768, k = 64: 8.3; 100 x 264 -> 352, k = 64: 8.7; 32 x 1024 -> 2048,
 // k = 128, 64 blocks of 64 KB: 9.2; 4 x 2048 -> 10000, k = 32, 157 blocks: 9.0; 64 x 768 -> 2048, k = 64, 128 blocks: 9.9.  At the line the
 // two are about even, whichever the host: 256 x 512 -> 640, k = 128, 160 blocks of 32 KB and 256 tags: 10.7 in bf16 and 11.6 in fp32, two launches
 // 9.3 and 9.7 on the fastest host, 11.7 and 11.5 in a program; 224 x 512 -> 640, k = 96, 140 blocks, 168 tags, bf16: 12.2, and 9.5 or 11.3.
 struct FewPlan {
-    int wave_values, chunks, ranges;
+    int wave_values, waves, chunks, ranges;   // waves: of a contracting block, and of both kinds where they are one launch
     int tile, tiles, tc, te;
     int c_blocks, e_blocks;
     bool sum, one;
@@ -512,13 +526,15 @@ static FewPlan few_plan(const rdb_linear_desc *d)
     const int64_t per_chunk = (int64_t)f.ranges * f.tile * FEW_COEFS * 4;   // of a tile
     f.sum = cdiv(d->in_f, chunk) * per_chunk * std::min(f.te, f.tiles) > 200 * 1024;
     if (f.sum && chunk > 256 && c_groups == 1) chunk = 256;
-    f.wave_values = (int)chunk / 4;
     f.chunks = (int)cdiv(d->in_f, chunk);
     f.part_bytes = f.chunks * per_chunk * f.tiles;
     f.c_blocks = (int)(f.chunks * f.ranges * c_groups);
     f.e_blocks = (int)(rows * cdiv(f.tiles, f.te));
     const int64_t block_bytes = f.chunks * per_chunk * std::min(f.te, f.tiles);   // what an expanding block reads
-    f.one = !f.sum && ((f.e_blocks <= 64 && block_bytes <= 100 * 1024) || (f.e_blocks <= 160 && block_bytes <= 32 * 1024));
+    f.one = !f.sum && ((f.e_blocks <= 64 && block_bytes <= 100 * 1024) || (f.e_blocks <= 160 && block_bytes <= 32 * 1024) ||
+                       (f.e_blocks <= 192 && block_bytes <= 16 * 1024 && f.c_blocks <= 32));
+    f.waves = (int)std::min<int64_t>(f.one ? (d->k <= 256 ? 8 : 4) : 16, chunk / 32);
+    f.wave_values = (int)chunk / f.waves;
     return f;
 }
 
@@ -569,16 +585,26 @@ int64_t linear_few_workspace(const rdb_linear_desc *d)
 
 template <typename E, int KS, int TC, int TE> static int few_launch(FewParams p, const FewPlan &f, int c_blocks, bool one, hipStream_t s)
 {
-    const size_t smem_z = (size_t)4 * TC * 1024, smem_y = (size_t)3 * TE * 16 * (KS * 32 + 8) * 2, smem = std::max(smem_z, smem_y);
-    const auto kernel = few_fwd_kernel<E, KS, TC, TE>;
-    if (int rc = reserve_lds(reinterpret_cast<const void *>(kernel), smem, "few_fwd_kernel")) return rc;
+    const size_t smem_y = (size_t)3 * TE * 16 * (KS * 32 + 8) * 2;
+    const auto fused = [&](auto waves_, size_t smem, unsigned blocks, const char *name) {
+        constexpr int WAVES = decltype(waves_)::value;
+        const auto kernel = few_fwd_kernel<E, KS, TC, TE, WAVES>;
+        if (int rc = reserve_lds(reinterpret_cast<const void *>(kernel), std::max((size_t)WAVES * TC * 1024, smem_y), name)) return rc;
+        kernel<<<blocks, WAVES * 64, smem, s>>>(p);
+        return check_launch(name);
+    };
+    typedef std::integral_constant<int, 4> W4;
+    typedef std::integral_constant<int, 8> W8;
     p.c_blocks = c_blocks;
     if (one) {
-        kernel<<<(unsigned)(c_blocks + f.e_blocks), 256, smem, s>>>(p);
-        return check_launch("few_fwd_kernel");
+        const unsigned blocks = (unsigned)(c_blocks + f.e_blocks);
+        const size_t smem = std::max((size_t)f.waves * TC * 1024, smem_y);
+        return f.waves == 8 ? fused(W8{}, smem, blocks, "few_fwd_kernel") : fused(W4{}, smem, blocks, "few_fwd_kernel");
     }
-    kernel<<<(unsigned)c_blocks, 256, smem_z, s>>>(p);
-    if (int rc = check_launch("few_fwd_kernel (z)")) return rc;
+    if (f.waves == 16) few_contract_kernel<E, TC, 16><<<(unsigned)c_blocks, 1024, 0, s>>>(p);
+    else if (f.waves == 8) few_contract_kernel<E, TC, 8><<<(unsigned)c_blocks, 512, 0, s>>>(p);
+    else few_contract_kernel<E, TC, 4><<<(unsigned)c_blocks, 256, 0, s>>>(p);
+    if (int rc = check_launch("few_contract_kernel")) return rc;
     if (f.sum) {
         const int64_t n4 = (int64_t)p.tiles * p.ranges * p.tile * 4;
         few_sum_kernel<<<(unsigned)cdiv(n4, 256), 256, 0, s>>>(p.part, n4, p.chunks);
@@ -586,8 +612,7 @@ template <typename E, int KS, int TC, int TE> static int few_launch(FewParams p,
         p.chunks = 1;
     }
     p.c_blocks = 0;
-    kernel<<<(unsigned)f.e_blocks, 256, smem_y, s>>>(p);
-    return check_launch("few_fwd_kernel (y)");
+    return fused(W4{}, smem_y, (unsigned)f.e_blocks, "few_fwd_kernel (y)");
 }
 template <typename E> static int few_dispatch(const FewParams &p, const FewPlan &f, int c_blocks, bool one, hipStream_t s)
 {

@@ -166,3 +166,11 @@ def test_a_wait_that_gives_up(T):
         hip.sync_check()
     hip.set_one_launch(1)
     assert torch.equal(hip.linear_fwd(x, c, in_f, out_f, in_f, 1, 5), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,in_f,out_f,k", [(3, 3990, 12300, 40), (20, 4095, 11000, 250), (1, 2047, 11010, 63), (8, 2049, 12287, 64), (9, 2048, 12290, 64), (64, 3000, 9000, 200),
+                                            (7, 1025, 4000, 300), (5, 500, 4000, 70), (2, 33, 20000, 9)])
+def test_chunks_in_eight_and_sixteen_waves(T, in_f, out_f, k, dtype):
+    """Four, eight or sixteen waves to a chunk, the last chunk's not all with something to add; both sides of the line to one launch."""
+    test_against_float64(T, in_f, out_f, k, dtype)

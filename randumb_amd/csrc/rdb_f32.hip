@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256) void f32_sum_scalars_kernel(float *__restrict_
 __global__ __launch_bounds__(256) void f32_sum_splits_kernel(FgSum a, FgSum b)
 {
     const bool second = (int)blockIdx.x >= a.blocks;
-    f32_sum_block(second ? b : a, (int)blockIdx.x - (second ? a.blocks : 0));
+    f32_sum_block(second ? b : a, (int)blockIdx.x - (second ? a.blocks : 0), threadIdx.x);
 }
 static FgSum fg_sum(void *out, int out_bf16, const float *part, int64_t n, int64_t stride, int splits, const float *bias = nullptr, int64_t cols = 0)
 {
@@ -159,8 +159,11 @@ static int fg_launch_ranges(FgProduct q, int room, float *part, int64_t stride, 
 
 // Two such products that do not need each other, in one launch, and their sums in one: t = dy . C and dC = dy^T . z.
 int fg_launch_pair(const FgProduct &t, const FgProduct &dc, hipStream_t s);   // rdb_f32_pair.hip
+// dc_sum: dC's sum where it is left to the launch that comes next, dx = t . N, whose blocks leave compute units free: where t's ranges are one, so that no launch of sums is left, or dC's
+// partial matrices are long enough, 8 MB, for a few of the product's blocks to lose less than that launch does.  2048 tokens x 768 -> 3072, k = 256, 16 MB: sums 7.6 -> 4.8 us,
+// dx 12.5 -> 13.2, step 98.3 -> 96.1; 4097 x 1001 -> 999, k = 100 in bf16, 6 MB: sums 4.5 -> 4.2, dx 15.6 -> 16.7 with dC's beside it.
 static int fg_launch_pair_ranges(FgProduct t, int t_room, float *t_part, int64_t t_stride, FgProduct dc, int dc_room, float *dc_part, int64_t dc_stride,
-                                 int num_cus, hipStream_t s)
+                                 int num_cus, hipStream_t s, FgSum &dc_sum)
 {
     const FgPairPlan plan = fg_plan_pair({t.M, dc.M}, {t.N, dc.N}, {t.K, dc.K}, num_cus, {t_room, dc_room}, t.a_es == 2);
     FgProduct *const q[2] = {&t, &dc};
@@ -181,7 +184,9 @@ static int fg_launch_pair_ranges(FgProduct t, int t_room, float *t_part, int64_t
         }
     }
     if (int rc = fg_launch_pair(t, dc, s)) return rc;
-    return fg_launch_sums(sum[0], sum[1], s);
+    const bool beside = !sum[0].blocks || sum[1].n * sum[1].splits * 4 >= (8 << 20);
+    dc_sum = beside ? sum[1] : FgSum{};
+    return fg_launch_sums(sum[0], beside ? FgSum{} : sum[1], s);
 }
 
 // What z's launch of sums counts for on the host in a training step, which has 60 to 70 us of host work (a forward pass alone has 10, and its kernels are what
@@ -270,10 +275,12 @@ static FgProduct fg_t(float *t, const void *dy, int64_t lddy, const void *coef, 
     return q;
 }
 // dx[T x in_f] = t . N: the B side's rows are input features, hashed
-static int fg_dx_from_t(void *dx, int64_t lddx, const float *t, const rdb_linear_desc *d, int num_cus, hipStream_t s)
+// sum: one that is still to be done, beside the product
+static int fg_dx_from_t(void *dx, int64_t lddx, const float *t, const rdb_linear_desc *d, int num_cus, hipStream_t s, const FgSum &sum = {})
 {
     FgProduct q = {t, d->k, d->tokens * d->k, nullptr, 0, 0, (float *)dx, lddx, nullptr, d->tokens, d->in_f, d->k, 0, 0, 0, 0, d->seed};
     q.out_bf16 = d->act_dtype == RDB_BF16;
+    q.sum = sum;
     return fg_launch<FG_KCONT, FG_NOISE_I>(q, num_cus, s, "f32_gemm_kernel (dx = t . N)");
 }
 // dC[out_f x k] = dy^T . z: both sides are read across their rows (the contraction runs over the tokens)
@@ -296,10 +303,11 @@ static int fg_backward(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, con
     if (dx && dcoef && f32_split_mode()) {
         float *t = (float *)workspace;
         const int64_t zt = up256(d->tokens * d->k * 4) / 4;
+        FgSum dc_sum;
         if (int rc = fg_launch_pair_ranges(fg_t(t, dy, lddy, coef, d), t_room(d, num_cus), t + zt, zt, fg_dc(dcoef, dcoef_dtype, dy, lddy, z, d),
-                                           room, dc_part, dc_stride, num_cus, s))
+                                           room, dc_part, dc_stride, num_cus, s, dc_sum))
             return rc;
-        return fg_dx_from_t(dx, lddx, t, d, num_cus, s);
+        return fg_dx_from_t(dx, lddx, t, d, num_cus, s, dc_sum);
     }
     if (dx) {
         if (int rc = linear_dx_f32(dx, lddx, dy, lddy, coef, nullptr, d, num_cus, workspace, workspace_bytes, s)) return rc;

@@ -2,6 +2,7 @@
 // launched.  Each rdb_f32_*.hip compiles the kernels of some pairs of operand sources (they build in parallel).
 #pragma once
 #include "rdb_gemm.hpp"
+#include "rdb_sums.hpp"
 #include <algorithm>
 #include <type_traits>
 
@@ -92,6 +93,8 @@ struct FgParams {
     int64_t lddot;
     float *dot_part;            // with dotm: one value per block, in block order (x fastest, then y)
     FgValues values;            // FG_NOISE_M on the B side: formed by the last blocks along z
+    FgSum sum;                  // FG_NOISE_I on the B side: a sum that an earlier launch left to do, by the last blocks along z
+    int sum_slices;
 };
 
 // fp32 products on the bf16 matrix cores.  v = h + m + l exactly, each part a bf16: v rounded to the nearest, what is left rounded to
@@ -744,6 +747,15 @@ __global__ __launch_bounds__(FG_THREADS * G, (fg_min_waves<BM, G, BSRC>())) void
             return;
         }
     }
+    if constexpr (BSRC == FG_NOISE_I) {
+        const unsigned products = gridDim.z - (unsigned)p.sum_slices;
+        if (blockIdx.z >= products) {
+            const int tiles = (int)(gridDim.x * gridDim.y), block = (int)(blockIdx.z - products) * tiles + (int)(blockIdx.y * gridDim.x + blockIdx.x);
+            const int mine = block * G + (int)threadIdx.x / FG_THREADS;
+            if (mine < p.sum.blocks) f32_sum_block(p.sum, mine, threadIdx.x & (FG_THREADS - 1));
+            return;
+        }
+    }
     f32_gemm_block<BM, G, ASRC, BSRC, EPI, VEC, SPLIT, AES, BES>(p, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, lds, not_finite);
 }
 
@@ -921,6 +933,7 @@ struct FgProduct {
     // fp32 matrix instructions (its unit-coefficient results are compared bit for bit)
     bool split = f32_split_mode() != 0;
     FgValues values = {};
+    FgSum sum = {};
 };
 
 #define FG_LAUNCH_GROUPS(BM_, G_, EPI_)                                                                               \
@@ -992,6 +1005,7 @@ inline FgParams fg_params(const FgProduct &q)
     p.lddot = q.lddot;
     p.dot_part = q.dot_part;
     p.values = q.values;
+    p.sum = q.sum;
     return p;
 }
 // 16-byte pieces (8 of a bf16 matrix: four values) when both matrices allow them: aligned bases and leading dimensions, and the extent
@@ -1014,12 +1028,13 @@ template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_
     }
     if (!fg_fits(q)) return RDB_E_UNSUPPORTED;
     if constexpr (BSRC == FG_NOISE_M) q.values.slices = fg_value_slices(q.values, cdiv(q.M, q.bm) * cdiv(q.N, FG_BN), FG_THREADS * (q.split ? q.groups : 1));
-    const FgParams p = fg_params(q);
+    FgParams p = fg_params(q);
     const int splits = (int)cdiv(q.K, p.kchunk);
+    if (BSRC == FG_NOISE_I) p.sum_slices = (int)cdiv(cdiv(q.sum.blocks, q.split ? q.groups : 1), cdiv(q.M, q.bm) * cdiv(q.N, FG_BN));
     const bool vec = fg_vec(q, ASRC, BSRC);
     const bool a16 = (ASRC == FG_KCONT || ASRC == FG_MCONT) && q.a_es == 2, b16 = (BSRC == FG_KCONT || BSRC == FG_MCONT) && q.b_es == 2;
     if (q.split && ((a16 && b16) ? !Groups::a16_b16 : a16 ? !Groups::a16_b32 : b16 && !Groups::a32_b16)) return RDB_E_UNSUPPORTED;
-    const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)(splits + (BSRC == FG_NOISE_M ? q.values.slices : 0)));
+    const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)(splits + (BSRC == FG_NOISE_M ? q.values.slices : 0) + p.sum_slices));
     auto run = [&](auto epi_) {
         constexpr int EPI = decltype(epi_)::value;
         if (q.bm == 128 && q.groups == 2) FG_LAUNCH_GROUPS(128, 2, EPI);

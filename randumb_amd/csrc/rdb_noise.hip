@@ -432,7 +432,7 @@ template <bool GATHER, int MT, int WM, bool LAYER> __global__ __launch_bounds__(
             return;
         }
         if (b >= p.main_blocks) {
-            f32_sum_block(p.sum, b - p.main_blocks);
+            f32_sum_block(p.sum, b - p.main_blocks, t);
             return;
         }
         by = b / p.mblocks;

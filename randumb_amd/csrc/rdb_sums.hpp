@@ -32,9 +32,9 @@ struct FgSum {
     uint32_t cols;
 };
 // block of q.blocks, of 256 threads
-__device__ __forceinline__ void f32_sum_block(const FgSum &q, int block)
+__device__ __forceinline__ void f32_sum_block(const FgSum &q, int block, int thread)
 {
-    const int64_t i = (int64_t)block * 256 + threadIdx.x, n4 = q.vec ? q.n / 4 : 0;
+    const int64_t i = (int64_t)block * 256 + thread, n4 = q.vec ? q.n / 4 : 0;
     if (i < n4) {
         f32x4 v = sum_in_order<f32x4>(q.part + i * 4, q.stride, q.splits);
         if (q.bias) {

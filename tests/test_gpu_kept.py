@@ -106,3 +106,27 @@ def test_both_products_over_dy_in_one_launch(T, in_f, out_f, k, dtype):
     assert torch.equal(dx, again[0]) and torch.equal(dc, again[1])
     assert _rel(torch.autograd.grad(y, leaves[:1], dy.cuda(), retain_graph=True)[0], dx.double().cpu()) < 2 * tol
     assert _rel(torch.autograd.grad(y, leaves[1:], dy.cuda())[0], dc.double().cpu()) < 2 * tol
+
+
+@pytest.mark.parametrize("dtype,T,in_f,out_f,k", [(torch.float32, 2048, 768, 3072, 256), (torch.float32, 3000, 520, 100, 60), (torch.float32, 5000, 33, 2100, 257),
+                                                  (torch.float32, 700, 40, 3000, 300), (torch.bfloat16, 4097, 301, 2999, 200), (torch.bfloat16, 3001, 77, 129, 50)])
+def test_sums_of_the_coefficients_gradient_beside_dx(dtype, T, in_f, out_f, k):
+    """Both sides of the line, dx of one tile and of many, in every kind of block; against float64."""
+    from randumb_amd import SillyLinear, hip
+
+    layer = SillyLinear(in_f, out_f, [k, k], [3, 4], bias=False, device="cuda", dtype=dtype, matrix_coef=True)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    with torch.no_grad():
+        layer.weight_coef.normal_(0.0, 1.0, generator=g)
+    x = torch.randn(T, in_f, generator=g, device="cuda").to(dtype).requires_grad_()
+    dy = torch.randn(T, out_f, generator=g, device="cuda").to(dtype)
+    y = layer(x)
+    dx, dc = torch.autograd.grad(y, [x, layer.weight_coef], dy)
+    N, x64 = hip.sq5_fill_2d(in_f, k, 3).double(), x.detach().double()
+    want_dx, want_dc = (dy.double() @ layer.weight_coef.detach().double()) @ N.t(), dy.double().t() @ (x64 @ N)
+    # fp32 sums; bf16: rounded once at the end
+    tol = 3e-6 if dtype is torch.float32 else 2.0**-8
+    for got, want in ((dx, want_dx), (dc, want_dc)):
+        assert float((got.double() - want).norm() / want.norm()) < tol
+    again = torch.autograd.grad(layer(x), [x, layer.weight_coef], dy)
+    assert torch.equal(again[0], dx) and torch.equal(again[1], dc)

@@ -67,6 +67,12 @@ typedef struct rdb_pseudo_bias {
     int64_t k;
     uint32_t seed;
 } rdb_pseudo_bias;
+/* Where its gradients go, fp32: dcoef k values, dscale one; NULL where not wanted. */
+typedef struct rdb_pseudo_bias_grad {
+    float *dcoef, *dscale;
+    int64_t k;
+    uint32_t seed;
+} rdb_pseudo_bias_grad;
 
 /* ------------------------------------------------------------------------------------------ materialise
  * Replaces: op rten::materialize_fwd + materialize_fwd_kernel (R.py:235-290, 371-381) and
@@ -424,6 +430,11 @@ int rdb_linear_bwd_kept(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, fl
                         int64_t lddy, const void *x, int64_t ldx, const void *kept, const void *coef,
                         const void *scale_bias, const rdb_linear_desc *desc, void *workspace, int64_t workspace_bytes,
                         void *stream);
+/* The same and rdb_bias_bwd of dy, in the same launches where dy is small; a workspace that is enough for either. */
+int rdb_linear_bwd_kept_pseudo_bias(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy,
+                                    int64_t lddy, const void *x, int64_t ldx, const void *kept, const void *coef,
+                                    const void *scale_bias, const rdb_pseudo_bias_grad *bias, const rdb_linear_desc *desc,
+                                    void *workspace, int64_t workspace_bytes, void *stream);
 
 /* For tools that time the two kernel launches of rdb_linear_bwd_projected one by one (no counterpart in the reference):
  * part 1 enqueues only the first launch (dy.C into the workspace and the partial sums of dcoef), part 2 only the second

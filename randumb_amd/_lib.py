@@ -77,6 +77,7 @@ EXPORTS = [
     "rdb_linear_fwd_kept_pseudo_bias",
     "rdb_linear_fwd_kept_ws",
     "rdb_linear_bwd_kept",
+    "rdb_linear_bwd_kept_pseudo_bias",
     "rdb_set_big_tiles",
     "rdb_set_f32_split",
     "rdb_set_one_launch",
@@ -95,6 +96,12 @@ EXPORTS = [
 ]
 
 ABI_VERSION = 8   # what this binding was written against (rdb_abi_version)
+
+
+class PseudoBiasGrad(ctypes.Structure):
+    """Mirror of ``rdb_pseudo_bias_grad``."""
+
+    _fields_ = [("dcoef", ctypes.c_void_p), ("dscale", ctypes.c_void_p), ("k", ctypes.c_int64), ("seed", ctypes.c_uint32)]
 
 
 class LinearDesc(ctypes.Structure):
@@ -235,6 +242,8 @@ def load() -> ctypes.CDLL:
     L.rdb_linear_fwd_kept_ws.restype = ci
     L.rdb_linear_bwd_kept.argtypes = [vp, i64, vp, ci, vp, vp, i64, vp, i64, vp, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_bwd_kept.restype = ci
+    L.rdb_linear_bwd_kept_pseudo_bias.argtypes = [vp, i64, vp, ci, vp, vp, i64, vp, i64, vp, vp, vp, vp, dp, vp, i64, vp]
+    L.rdb_linear_bwd_kept_pseudo_bias.restype = ci
     L.rdb_set_big_tiles.argtypes = [ci]
     L.rdb_set_big_tiles.restype = ci
     L.rdb_set_f32_split.argtypes = [ci]

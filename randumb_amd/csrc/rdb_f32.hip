@@ -275,12 +275,13 @@ static FgProduct fg_t(float *t, const void *dy, int64_t lddy, const void *coef, 
     return q;
 }
 // dx[T x in_f] = t . N: the B side's rows are input features, hashed
-// sum: one that is still to be done, beside the product
-static int fg_dx_from_t(void *dx, int64_t lddx, const float *t, const rdb_linear_desc *d, int num_cus, hipStream_t s, const FgSum &sum = {})
+// sum, bias: what is still to be done, beside the product
+static int fg_dx_from_t(void *dx, int64_t lddx, const float *t, const rdb_linear_desc *d, int num_cus, hipStream_t s, const FgSum &sum = {}, const BiasGrad &bias = {})
 {
     FgProduct q = {t, d->k, d->tokens * d->k, nullptr, 0, 0, (float *)dx, lddx, nullptr, d->tokens, d->in_f, d->k, 0, 0, 0, 0, d->seed};
     q.out_bf16 = d->act_dtype == RDB_BF16;
     q.sum = sum;
+    q.bias_grad = bias;
     return fg_launch<FG_KCONT, FG_NOISE_I>(q, num_cus, s, "f32_gemm_kernel (dx = t . N)");
 }
 // dC[out_f x k] = dy^T . z: both sides are read across their rows (the contraction runs over the tokens)
@@ -294,9 +295,9 @@ static FgProduct fg_dc(void *dcoef, int dcoef_dtype, const void *dy, int64_t ldd
 }
 int linear_dx_f32(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *coef, const void *scale_bias, const rdb_linear_desc *d,
                   int num_cus, void *workspace, int64_t workspace_bytes, hipStream_t s);
-// dx and / or dC (each NULL where it is not wanted) from dy, z and C; dc_part: room for dC's partial matrices
+// dx and / or dC (each NULL where it is not wanted) from dy, z and C; dc_part: room for dC's partial matrices; bias: a gradient from dy that the last launch carries
 static int fg_backward(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, const void *dy, int64_t lddy, const float *z, const void *coef,
-                       const rdb_linear_desc *d, int num_cus, void *workspace, int64_t workspace_bytes, float *dc_part, hipStream_t s)
+                       const rdb_linear_desc *d, int num_cus, void *workspace, int64_t workspace_bytes, float *dc_part, hipStream_t s, const BiasGrad &bias = {})
 {
     const int room = dc_room(d, num_cus);
     const int64_t dc_stride = up256(d->out_f * d->k * 4) / 4;
@@ -307,13 +308,15 @@ static int fg_backward(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, con
         if (int rc = fg_launch_pair_ranges(fg_t(t, dy, lddy, coef, d), t_room(d, num_cus), t + zt, zt, fg_dc(dcoef, dcoef_dtype, dy, lddy, z, d),
                                            room, dc_part, dc_stride, num_cus, s, dc_sum))
             return rc;
-        return fg_dx_from_t(dx, lddx, t, d, num_cus, s, dc_sum);
+        return fg_dx_from_t(dx, lddx, t, d, num_cus, s, dc_sum, bias);
     }
     if (dx) {
         if (int rc = linear_dx_f32(dx, lddx, dy, lddy, coef, nullptr, d, num_cus, workspace, workspace_bytes, s)) return rc;
     }
-    if (!dcoef) return RDB_OK;
-    return fg_launch_ranges<FG_MCONT, FG_MCONT>(fg_dc(dcoef, dcoef_dtype, dy, lddy, z, d), room, dc_part, dc_stride, num_cus, s, "f32_gemm_kernel (dC = dy^T . z)");
+    if (!dcoef) return bias.blocks ? bias_direct_launch(bias, s) : RDB_OK;
+    FgProduct dc = fg_dc(dcoef, dcoef_dtype, dy, lddy, z, d);
+    dc.bias_grad = bias;
+    return fg_launch_ranges<FG_MCONT, FG_MCONT>(dc, room, dc_part, dc_stride, num_cus, s, "f32_gemm_kernel (dC = dy^T . z)");
 }
 
 int linear_dx_f32(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *coef, const void *scale_bias, const rdb_linear_desc *d,
@@ -489,7 +492,7 @@ __global__ __launch_bounds__(256) void f32_rbias_sum_kernel(bf16_t *__restrict__
 // comes out of the random-bias product that dx needs anyway.
 int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x, int64_t ldx,
                         const void *kept, const void *coef, const void *scale_bias, const rdb_linear_desc *d, int num_cus, void *workspace,
-                        int64_t workspace_bytes, hipStream_t s)
+                        int64_t workspace_bytes, hipStream_t s, const BiasGrad &bias)
 {
     if (!linear_kept_f32_bytes(d) || !fg_aligned16(kept) || !workspace || !fg_aligned16(workspace) ||
         workspace_bytes < linear_bwd_kept_f32_workspace(d, num_cus) || d->tokens * lddy >= (1ll << 29) || (dx && d->tokens * lddx >= (1ll << 29)) ||
@@ -499,7 +502,7 @@ int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, fl
     const int r = dc_room(d, num_cus);
     float *const dots = reinterpret_cast<float *>(dc_part + (r > 1 ? (int64_t)r * up256(d->out_f * d->k * 4) : 0));
     if (int rc = fg_backward(dx, lddx, dcoef, dcoef_dtype, dy, lddy, static_cast<const float *>(kept), coef, d, num_cus, workspace, workspace_bytes,
-                             reinterpret_cast<float *>(dc_part), s))
+                             reinterpret_cast<float *>(dc_part), s, bias))
         return rc;
     if (!scale_bias || (!dx && !d_scale_bias)) return RDB_OK;
     FgProduct q;

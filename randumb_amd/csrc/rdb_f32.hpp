@@ -1,6 +1,7 @@
 // Products at fp32 accuracy on the matrix cores: the kernel template of rdb_f32.hip, how a product is planned and how it is
 // launched.  Each rdb_f32_*.hip compiles the kernels of some pairs of operand sources (they build in parallel).
 #pragma once
+#include "rdb_bias.hpp"
 #include "rdb_gemm.hpp"
 #include "rdb_sums.hpp"
 #include <algorithm>
@@ -95,6 +96,8 @@ struct FgParams {
     FgValues values;            // FG_NOISE_M on the B side: formed by the last blocks along z
     FgSum sum;                  // FG_NOISE_I on the B side: a sum that an earlier launch left to do, by the last blocks along z
     int sum_slices;
+    BiasGrad bias_grad;         // FG_NOISE_I on the B side, or two FG_MCONT: by the blocks before those
+    int bias_slices;
 };
 
 // fp32 products on the bf16 matrix cores.  v = h + m + l exactly, each part a bf16: v rounded to the nearest, what is left rounded to
@@ -733,6 +736,9 @@ template <int BM, int G, int BSRC> constexpr int fg_min_waves()
     if (G == 1) return BM == 128 && BSRC == FG_NOISE_1D ? 3 : 2;
     return G == 2 && BM == 64 && (BSRC == FG_NOISE_M || BSRC == FG_NOISE_I) ? 4 : 1;
 }
+// The last launch of a backward pass, dx = t . N or dC = dy^T . z alone, carries the gradient of a pseudorandom bias where dy is small: a launch of its own is 6 us
+// of kernel and as much on the host (128 images through 784 -> 256 -> 10, k = 64, fp32: 18 launches a step, 16 without).
+constexpr bool fg_carries_bias(int asrc, int bsrc) { return bsrc == FG_NOISE_I || (asrc == FG_MCONT && bsrc == FG_MCONT); }
 template <int BM, int G, int ASRC, int BSRC, int EPI, bool VEC, bool SPLIT, int AES, int BES>
 __global__ __launch_bounds__(FG_THREADS * G, (fg_min_waves<BM, G, BSRC>())) void f32_gemm_kernel(FgParams p)
 {
@@ -747,12 +753,18 @@ __global__ __launch_bounds__(FG_THREADS * G, (fg_min_waves<BM, G, BSRC>())) void
             return;
         }
     }
-    if constexpr (BSRC == FG_NOISE_I) {
-        const unsigned products = gridDim.z - (unsigned)p.sum_slices;
+    if constexpr (fg_carries_bias(ASRC, BSRC)) {
+        const unsigned sums = gridDim.z - (unsigned)p.sum_slices, products = sums - (unsigned)p.bias_slices;
         if (blockIdx.z >= products) {
-            const int tiles = (int)(gridDim.x * gridDim.y), block = (int)(blockIdx.z - products) * tiles + (int)(blockIdx.y * gridDim.x + blockIdx.x);
-            const int mine = block * G + (int)threadIdx.x / FG_THREADS;
-            if (mine < p.sum.blocks) f32_sum_block(p.sum, mine, threadIdx.x & (FG_THREADS - 1));
+            const bool sum = BSRC == FG_NOISE_I && blockIdx.z >= sums;
+            const int tiles = (int)(gridDim.x * gridDim.y), block = (int)(blockIdx.z - (sum ? sums : products)) * tiles + (int)(blockIdx.y * gridDim.x + blockIdx.x);
+            if (sum) {
+                const int mine = block * G + (int)threadIdx.x / FG_THREADS;
+                if (mine < p.sum.blocks) f32_sum_block(p.sum, mine, threadIdx.x & (FG_THREADS - 1));
+            } else if (block < p.bias_grad.blocks) {
+                if (p.bias_grad.bf16) bias_direct_block<bf16_t, FG_THREADS * G>(p.bias_grad, block, lds);
+                else bias_direct_block<float, FG_THREADS * G>(p.bias_grad, block, lds);
+            }
             return;
         }
     }
@@ -934,6 +946,7 @@ struct FgProduct {
     bool split = f32_split_mode() != 0;
     FgValues values = {};
     FgSum sum = {};
+    BiasGrad bias_grad = {};   // bias_direct holds for it
 };
 
 #define FG_LAUNCH_GROUPS(BM_, G_, EPI_)                                                                               \
@@ -1006,6 +1019,7 @@ inline FgParams fg_params(const FgProduct &q)
     p.dot_part = q.dot_part;
     p.values = q.values;
     p.sum = q.sum;
+    p.bias_grad = q.bias_grad;
     return p;
 }
 // 16-byte pieces (8 of a bf16 matrix: four values) when both matrices allow them: aligned bases and leading dimensions, and the extent
@@ -1030,11 +1044,18 @@ template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_
     if constexpr (BSRC == FG_NOISE_M) q.values.slices = fg_value_slices(q.values, cdiv(q.M, q.bm) * cdiv(q.N, FG_BN), FG_THREADS * (q.split ? q.groups : 1));
     FgParams p = fg_params(q);
     const int splits = (int)cdiv(q.K, p.kchunk);
-    if (BSRC == FG_NOISE_I) p.sum_slices = (int)cdiv(cdiv(q.sum.blocks, q.split ? q.groups : 1), cdiv(q.M, q.bm) * cdiv(q.N, FG_BN));
+    const int64_t tiles = cdiv(q.M, q.bm) * cdiv(q.N, FG_BN);
+    const int groups = q.split ? q.groups : 1;
+    if (BSRC == FG_NOISE_I) p.sum_slices = (int)cdiv(cdiv(q.sum.blocks, groups), tiles);
+    if (fg_carries_bias(ASRC, BSRC) && q.bias_grad.blocks) {
+        const BiasGrad &g = q.bias_grad;
+        if (bias_direct(g.rows, g.n, g.bf16 ? 2 : 4, g.k, num_cus, FG_THREADS * groups)) p.bias_slices = (int)cdiv(g.blocks, tiles);
+        else if (int rc = bias_direct_launch(g, s)) return rc;   // too few threads to a block
+    }
     const bool vec = fg_vec(q, ASRC, BSRC);
     const bool a16 = (ASRC == FG_KCONT || ASRC == FG_MCONT) && q.a_es == 2, b16 = (BSRC == FG_KCONT || BSRC == FG_MCONT) && q.b_es == 2;
     if (q.split && ((a16 && b16) ? !Groups::a16_b16 : a16 ? !Groups::a16_b32 : b16 && !Groups::a32_b16)) return RDB_E_UNSUPPORTED;
-    const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)(splits + (BSRC == FG_NOISE_M ? q.values.slices : 0) + p.sum_slices));
+    const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)(splits + (BSRC == FG_NOISE_M ? q.values.slices : 0) + p.sum_slices + p.bias_slices));
     auto run = [&](auto epi_) {
         constexpr int EPI = decltype(epi_)::value;
         if (q.bm == 128 && q.groups == 2) FG_LAUNCH_GROUPS(128, 2, EPI);

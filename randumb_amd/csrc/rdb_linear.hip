@@ -11,6 +11,7 @@
 // RandumbTensorConstructor.backward -> materialize_bwd / scale_bias_bwd (RandumbTensor.py:979-990).
 #include <algorithm>
 
+#include "rdb_bias.hpp"
 #include "rdb_blocks.hpp"
 #include "rdb_tile.hpp"
 
@@ -1397,7 +1398,7 @@ int linear_fwd_kept_f32(void *y, int64_t ldy, void *kept, const void *x, int64_t
                         const rdb_linear_desc *d, int num_cus, void *scratch, int64_t scratch_bytes, hipStream_t s);
 int linear_bwd_kept_f32(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x, int64_t ldx,
                         const void *kept, const void *coef, const void *scale_bias, const rdb_linear_desc *d, int num_cus, void *workspace,
-                        int64_t workspace_bytes, hipStream_t s);
+                        int64_t workspace_bytes, hipStream_t s, const BiasGrad &bias);
 }
 
 static bool kept_layer(const rdb_linear_desc *d)
@@ -1446,23 +1447,54 @@ extern "C" int rdb_linear_fwd_kept_ws(void *y, int64_t ldy, void *kept, const vo
     return fwd_kept(who, y, ldy, kept, x, ldx, coef, scale_bias, bias, pseudo_bias, d, workspace, workspace_bytes, stream);
 }
 
+static int bwd_kept(const char *who, void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x, int64_t ldx,
+                    const void *kept, const void *coef, const void *scale_bias, const rdb_pseudo_bias_grad *bias, const rdb_linear_desc *d, void *workspace,
+                    int64_t workspace_bytes, void *stream)
+{
+    if (int rc = check_desc(who, d)) return rc;
+    if (!kept_layer(d)) return set_error(RDB_E_UNSUPPORTED, "%s: a layer of which nothing is kept (rdb_linear_kept_bytes)", who);
+    if (!dy || (dx && !coef) || (dcoef && !kept) || (d_scale_bias && (!x || !scale_bias)))
+        return set_error(RDB_E_NULL, "%s: dy, x, kept, coef or scale_bias is NULL", who);
+    if (lddy < d->out_f || (dx && lddx < d->in_f) || (d_scale_bias && ldx < d->in_f))
+        return set_error(RDB_E_SHAPE, "%s: leading dimension smaller than the row", who);
+    if (dcoef_dtype != RDB_F32 && dcoef_dtype != RDB_BF16) return set_error(RDB_E_DTYPE, "%s: unknown dcoef dtype %d", who, dcoef_dtype);
+    BiasGrad g = {};
+    bool apart = false;   // the bias's gradient is two launches of its own
+    if (bias) {
+        if (bias->k < 0) return set_error(RDB_E_SHAPE, "%s: a bias of %lld coefficients", who, (long long)bias->k);
+        if (workspace_bytes < rdb_bias_bwd_workspace_bytes(d->tokens, d->out_f))
+            return set_error(RDB_E_WORKSPACE, "%s: workspace of %lld bytes needed, %lld given", who, (long long)rdb_bias_bwd_workspace_bytes(d->tokens, d->out_f),
+                             (long long)workspace_bytes);
+        const bool wanted = (bias->dcoef && bias->k > 0) || bias->dscale;
+        apart = wanted && !(bias_direct(d->tokens, d->out_f, d->act_dtype == RDB_BF16 ? 2 : 4, bias->k, num_compute_units()) && (dx || dcoef || d_scale_bias));
+        if (wanted && !apart)
+            g = {bias->k > 0 ? bias->dcoef : nullptr, bias->dscale, dy, lddy, bias->k, (int)d->tokens, (int)d->out_f, d->act_dtype == RDB_BF16, bias->seed,
+                 (int)((bias->dcoef ? cdiv(bias->k, BIAS_M) : 0) + (bias->dscale ? 1 : 0))};
+    }
+    int rc = linear_bwd_kept_f32(dx, lddx, dcoef, dcoef_dtype, d_scale_bias, dy, lddy, x, ldx, kept, coef, scale_bias, d, num_compute_units(), workspace, workspace_bytes,
+                                 (hipStream_t)stream, g);
+    if (rc == RDB_E_UNSUPPORTED)
+        return set_error(rc, "%s: needs a 16-byte aligned workspace of rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_KEPT) bytes and tokens times each leading dimension "
+                             "below 2^29", who);
+    if (!rc && apart)
+        rc = rdb_bias_bwd(bias->dcoef, bias->dscale, dy, d->act_dtype, lddy, d->tokens, d->out_f, bias->k, bias->seed, workspace, workspace_bytes, stream);
+    return rc;
+}
+
 extern "C" int rdb_linear_bwd_kept(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x,
                                    int64_t ldx, const void *kept, const void *coef, const void *scale_bias, const rdb_linear_desc *d, void *workspace,
                                    int64_t workspace_bytes, void *stream)
 {
-    if (int rc = check_desc("rdb_linear_bwd_kept", d)) return rc;
-    if (!kept_layer(d)) return set_error(RDB_E_UNSUPPORTED, "rdb_linear_bwd_kept: a layer of which nothing is kept (rdb_linear_kept_bytes)");
-    if (!dy || (dx && !coef) || (dcoef && !kept) || (d_scale_bias && (!x || !scale_bias)))
-        return set_error(RDB_E_NULL, "rdb_linear_bwd_kept: dy, x, kept, coef or scale_bias is NULL");
-    if (lddy < d->out_f || (dx && lddx < d->in_f) || (d_scale_bias && ldx < d->in_f))
-        return set_error(RDB_E_SHAPE, "rdb_linear_bwd_kept: leading dimension smaller than the row");
-    if (dcoef_dtype != RDB_F32 && dcoef_dtype != RDB_BF16) return set_error(RDB_E_DTYPE, "rdb_linear_bwd_kept: unknown dcoef dtype %d", dcoef_dtype);
-    const int rc = linear_bwd_kept_f32(dx, lddx, dcoef, dcoef_dtype, d_scale_bias, dy, lddy, x, ldx, kept, coef, scale_bias, d, num_compute_units(), workspace,
-                                       workspace_bytes, (hipStream_t)stream);
-    if (rc == RDB_E_UNSUPPORTED)
-        return set_error(rc, "rdb_linear_bwd_kept: needs a 16-byte aligned workspace of rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_KEPT) bytes and tokens "
-                             "times each leading dimension below 2^29");
-    return rc;
+    return bwd_kept("rdb_linear_bwd_kept", dx, lddx, dcoef, dcoef_dtype, d_scale_bias, dy, lddy, x, ldx, kept, coef, scale_bias, nullptr, d, workspace, workspace_bytes, stream);
+}
+
+extern "C" int rdb_linear_bwd_kept_pseudo_bias(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, float *d_scale_bias, const void *dy, int64_t lddy, const void *x,
+                                               int64_t ldx, const void *kept, const void *coef, const void *scale_bias, const rdb_pseudo_bias_grad *bias,
+                                               const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
+{
+    if (!bias) return set_error(RDB_E_NULL, "rdb_linear_bwd_kept_pseudo_bias: bias is NULL");
+    return bwd_kept("rdb_linear_bwd_kept_pseudo_bias", dx, lddx, dcoef, dcoef_dtype, d_scale_bias, dy, lddy, x, ldx, kept, coef, scale_bias, bias, d, workspace,
+                    workspace_bytes, stream);
 }
 
 // rdb_factored.hip, rdb_few.hip, rdb_smallk.hip

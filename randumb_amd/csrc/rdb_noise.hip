@@ -1,6 +1,7 @@
 // Noise probes, materialise forward/backward, random-bias gradient and embedding gather for gfx950.
 // These are the HBM-facing ops of the pseudorandom tensor (the fused linear kernels live in rdb_linear.hip).
 #include "rdb_common.hpp"
+#include "rdb_bias.hpp"
 #include "rdb_sums.hpp"
 #include <algorithm>
 #include <type_traits>
@@ -326,9 +327,7 @@ __device__ __forceinline__ double block_sum_ll(long long v, long long *scratch)
 }
 
 // ----------------------------------------------------------------------------------------------- column sums
-constexpr int BIAS_M = 4, BIAS_MAX_CHUNKS = 16;
-__device__ __forceinline__ float to_f32(float v) { return v; }
-__device__ __forceinline__ float to_f32(bf16_t v) { return bf16_to_f32(v); }
+constexpr int BIAS_MAX_CHUNKS = 16;
 static int bias_chunks(int64_t rows) { return (int)std::min<int64_t>(BIAS_MAX_CHUNKS, std::max<int64_t>(1, cdiv(rows, 32))); }
 
 // block (bx, by): 64 V columns of a chunk of rows; sh: 256 V floats
@@ -959,80 +958,23 @@ extern "C" int rdb_embed_bwd(float *dcoef, const int64_t *idx, int64_t n_idx, co
 // ----------------------------------------------------------------------------------------------- gradient of a pseudorandom bias
 // b[o] = sum_m noise(PRIME*o + m) coef[m] + s noise1d(o), added to every row of y: with g[o] = sum_t dy[t, o],
 // dcoef[m] = sum_o g[o] noise(PRIME*o + m) and ds = sum_o g[o] noise1d(o).
-// A small dy: one launch (bias_grad_direct_kernel).  Otherwise two.  First launch: the column sums of dy, a chunk of rows per block (memory-bound: dy is read once, 16 bytes a lane where its rows
+// A small dy: one launch (bias_grad_direct_kernel) or blocks of a layer's (rdb_bias.hpp).  Otherwise two.  First launch: the column sums of dy, a chunk of rows per block (memory-bound: dy is read once, 16 bytes a lane where its rows
 // allow), partial sums [chunks x n].  Second launch: every block adds the chunks up again for itself (a few rows out of L2)
 // and contracts them with the noise of its own BIAS_M coefficients; the n * k hashes are few.  Fixed orders throughout.
 // Replaces a column sum by the library, its cast, the contraction and the sum over its splits: 128 tokens x 256, k = 64: 12.6 ->
 // 6.0 us; 1024 tokens x 3072, k = 256: 19 -> 12 us.
 namespace rdb {
 
-// What a block of the gradient does with a column's sum g (block b: coefficients b * BIAS_M .. + 3; the block behind the last
-// coefficient: the scale), and at the end with its threads' shares.
-__device__ __forceinline__ void bias_contract(float (&acc)[BIAS_M], float g, uint32_t o, int64_t m0, bool scale, uint32_t seed)
+template <typename T> __global__ __launch_bounds__(1024) void bias_grad_direct_kernel(BiasGrad q)
 {
-    if (scale) {
-        acc[0] = fmaf(g, noise1d(o, seed), acc[0]);
-    } else {
-        const uint32_t f = sq5_first(o, (uint32_t)m0, seed);
-#pragma unroll
-        for (int j = 0; j < BIAS_M; ++j) acc[j] = fmaf(g, sq5_unit(sq5_tail(f + (uint32_t)j * SQ5_N1)), acc[j]);
-    }
+    __shared__ float sh[BIAS_M * 1024 / 64];
+    bias_direct_block<T, 1024>(q, blockIdx.x, sh);
 }
-template <int THREADS> __device__ __forceinline__ void bias_finish(float (&acc)[BIAS_M], float *dcoef, float *ds, int64_t m0, int64_t k, bool scale)
+int bias_direct_launch(const BiasGrad &q, hipStream_t s)
 {
-    __shared__ float sh[BIAS_M][THREADS / 64];
-#pragma unroll
-    for (int j = 0; j < BIAS_M; ++j) {
-#pragma unroll
-        for (int w = 32; w >= 1; w >>= 1) acc[j] += __shfl_xor(acc[j], w);
-        if ((threadIdx.x & 63) == 0) sh[j][threadIdx.x >> 6] = acc[j];
-    }
-    __syncthreads();
-    const int j = threadIdx.x;
-    if (j >= BIAS_M) return;
-    float v = 0.0f;
-#pragma unroll
-    for (int w = 0; w < THREADS / 64; w += 4) v += (sh[j][w] + sh[j][w + 1]) + (sh[j][w + 2] + sh[j][w + 3]);
-    if (scale) {
-        if (j == 0) ds[0] = v;
-    } else if (m0 + j < k) {
-        dcoef[m0 + j] = v;
-    }
-}
-
-// The whole gradient in one launch, for a dy so small that every block may read it: blocks of 1024 threads, as many of them side by side
-// on a column's rows as its outputs leave room for, sixteen rows in flight each.  3.3 us and 1.3 for every sixteen rows of a thread, against
-// 8.2 (and a launch more on the host) for the two: 128 rows x 256 5.9, 128 x 10 4.6, 512 x 128 8.5; 250 x 262, six turns, 11.0.  Only while a
-// compute unit has one block, which reads all of dy, whichever gradients are wanted (512 x 128: k = 1016 8.7, 1024 13.2, 4096 29.5, 16384 94, and the two
-// launches there 6.0, 6.0, 6.3 and 10 behind one another).
-constexpr int64_t BIAS_DIRECT_BYTES = 256 << 10, BIAS_DIRECT_TURNS = 4;
-constexpr int BIAS_AHEAD = 16;
-static int bias_wide(int64_t n) { return n < 1024 ? (int)cdiv(n, 64) * 64 : 1024; }   // threads along the outputs
-static bool bias_direct(int64_t rows, int64_t n, int es, int64_t k)
-{
-    if (rows <= 0 || n <= 0 || rows * n * es > BIAS_DIRECT_BYTES || cdiv(k, BIAS_M) + 1 > num_compute_units()) return false;
-    const int wide = bias_wide(n);
-    return cdiv(rows, BIAS_AHEAD * (1024 / wide)) * cdiv(n, wide) <= BIAS_DIRECT_TURNS;
-}
-template <typename T> __global__ __launch_bounds__(1024) void bias_grad_direct_kernel(float *__restrict__ dcoef, float *__restrict__ ds, const T *__restrict__ dy,
-                                                                                     int64_t ldy, int rows, int n, int wide, int64_t k, uint32_t seed)
-{
-    const int64_t m0 = (int64_t)blockIdx.x * BIAS_M;
-    const bool scale = !dcoef || m0 >= k;
-    const int beside = 1024 / wide, first = (int)threadIdx.x / wide;
-    float acc[BIAS_M] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int o = (int)threadIdx.x - first * wide; o < n && first < beside; o += wide) {
-        float g = 0.0f;
-        for (int r0 = first; r0 < rows; r0 += BIAS_AHEAD * beside) {
-            float v[BIAS_AHEAD];
-#pragma unroll
-            for (int i = 0; i < BIAS_AHEAD; ++i) v[i] = to_f32(dy[(int64_t)min(r0 + i * beside, rows - 1) * ldy + o]);   // clamped: loaded, not added
-#pragma unroll
-            for (int i = 0; i < BIAS_AHEAD; ++i) g += r0 + i * beside < rows ? v[i] : 0.0f;
-        }
-        bias_contract(acc, g, (uint32_t)o, m0, scale, seed);
-    }
-    bias_finish<1024>(acc, dcoef, ds, m0, k, scale);
+    if (q.bf16) bias_grad_direct_kernel<bf16_t><<<(unsigned)q.blocks, 1024, 0, s>>>(q);
+    else bias_grad_direct_kernel<float><<<(unsigned)q.blocks, 1024, 0, s>>>(q);
+    return check_launch("bias_grad_direct_kernel");
 }
 
 // The second launch.  THREADS: a thread's outputs are a chain of
@@ -1055,7 +997,8 @@ __device__ __forceinline__ void bias_grad_block(float *__restrict__ dcoef, float
         }
         bias_contract(acc, g, (uint32_t)o, m0, scale, seed);
     }
-    bias_finish<THREADS>(acc, dcoef, ds, m0, k, scale);
+    __shared__ float sh[BIAS_M * THREADS / 64];
+    bias_finish<THREADS>(acc, dcoef, ds, m0, k, scale, sh);
 }
 template <int THREADS> __global__ __launch_bounds__(THREADS) void bias_grad_kernel(float *__restrict__ dcoef, float *__restrict__ ds, const float *__restrict__ part, int chunks, int64_t n, int64_t k,
                                                        uint32_t seed)
@@ -1091,12 +1034,8 @@ extern "C" int rdb_bias_bwd(float *dcoef, float *ds, const void *dy, int dtype, 
     if (n > 0 && (!workspace || ((uintptr_t)workspace & 3) || workspace_bytes < rdb_bias_bwd_workspace_bytes(rows, n)))
         return set_error(RDB_E_WORKSPACE, "rdb_bias_bwd: workspace of %lld bytes needed, %lld given", (long long)rdb_bias_bwd_workspace_bytes(rows, n),
                          (long long)workspace_bytes);
-    if (bias_direct(rows, n, dtype == RDB_BF16 ? 2 : 4, k)) {
-        const int wide = bias_wide(n);
-        if (dtype == RDB_BF16) bias_grad_direct_kernel<bf16_t><<<(unsigned)blocks, 1024, 0, s>>>(dcoef, ds, static_cast<const bf16_t *>(dy), ldy, (int)rows, (int)n, wide, k, seed);
-        else bias_grad_direct_kernel<float><<<(unsigned)blocks, 1024, 0, s>>>(dcoef, ds, static_cast<const float *>(dy), ldy, (int)rows, (int)n, wide, k, seed);
-        return check_launch("bias_grad_direct_kernel");
-    }
+    if (bias_direct(rows, n, dtype == RDB_BF16 ? 2 : 4, k, num_compute_units()))
+        return bias_direct_launch({dcoef, ds, dy, ldy, k, (int)rows, (int)n, dtype == RDB_BF16, seed, (int)blocks}, s);
     if (n > 0) {
         const int64_t per = cdiv(rows, chunks);
         const int es = dtype == RDB_BF16 ? 2 : 4, V = 16 / es;

@@ -237,6 +237,25 @@ struct Bias {
         return {coef ? coef->numel() : -1, seed, coef ? (int64_t)coef->scalar_type() : 0, scale ? (int64_t)scale->scalar_type() : -1};
     }
 };
+// The gradients of a pseudorandom bias in fp32, as a call of the library takes them (none wanted: ref.k < 0), and in the bias's dtypes
+struct BiasGrads {
+    Tensor dc, ds;
+    rdb_pseudo_bias_grad ref = {nullptr, nullptr, -1, 0};
+    BiasGrads(AutogradContext *ctx, const Tensor &dy, const std::vector<int64_t> &m, int at)
+    {
+        if (m[0] < 0 || m[1] < 0) return;
+        const bool want_c = ctx->needs_input_grad(at), want_s = m[3] >= 0 && ctx->needs_input_grad(at + 1);
+        if (!want_c && !want_s) return;
+        const auto f32 = dy.options().dtype(at::kFloat);
+        if (want_c) dc = at::empty({m[0]}, f32);
+        if (want_s) ds = at::empty({1}, f32);
+        ref = {want_c ? dc.data_ptr<float>() : nullptr, want_s ? ds.data_ptr<float>() : nullptr, m[0], (uint32_t)m[1]};
+    }
+    std::pair<Tensor, Tensor> done(const std::vector<int64_t> &m) const
+    {
+        return {dc.defined() ? dc.to((at::ScalarType)m[2]) : Tensor(), ds.defined() ? ds.to((at::ScalarType)m[3]) : Tensor()};
+    }
+};
 // (gradient of the bias or its coefficients, gradient of its scale) from the column sums of dy; `at` is the bias's index among the
 // function's tensor inputs
 std::pair<Tensor, Tensor> bias_grads(AutogradContext *ctx, const Tensor &dy0, const std::vector<int64_t> &m, int at)
@@ -246,17 +265,14 @@ std::pair<Tensor, Tensor> bias_grads(AutogradContext *ctx, const Tensor &dy0, co
     if (!want_c && !want_s) return {};
     if (m[1] < 0) return {dy0.sum(0).to((at::ScalarType)m[2]), Tensor()};
     const Tensor dy = act(dy0);
-    const auto f32 = dy.options().dtype(at::kFloat);
-    Tensor dc = want_c ? at::empty({m[0]}, f32) : Tensor(), ds = want_s ? at::empty({1}, f32) : Tensor();
+    const c10::OptionalDeviceGuard guard(dy.device());
+    const BiasGrads g(ctx, dy, m, at);
     const int64_t need = rdb_bias_bwd_workspace_bytes(dy.size(0), dy.size(1));
     const Tensor ws = bytes(need, dy);
-    const c10::OptionalDeviceGuard guard(dy.device());
-    check(rdb_bias_bwd(want_c ? dc.data_ptr<float>() : nullptr, want_s ? ds.data_ptr<float>() : nullptr, dy.data_ptr(), code(dy.scalar_type()), dy.stride(0),
-                       dy.size(0), dy.size(1), m[0], (uint32_t)m[1], ptr(ws), need, stream_of(dy)),
+    check(rdb_bias_bwd(g.ref.dcoef, g.ref.dscale, dy.data_ptr(), code(dy.scalar_type()), dy.stride(0), dy.size(0), dy.size(1), g.ref.k, g.ref.seed, ptr(ws), need,
+                       stream_of(dy)),
           "rdb_bias_bwd");
-    if (want_c) dc = dc.to((at::ScalarType)m[2]);
-    if (want_s) ds = ds.to((at::ScalarType)m[3]);
-    return {dc, ds};
+    return g.done(m);
 }
 
 // ----------------------------------------------------------------------------------------------- the library's calls
@@ -437,10 +453,23 @@ class OneCallLinear : public Function<OneCallLinear> {
                 if (want_dx) dx = at::empty({dy.size(0), l.in_f}, dy.options());
                 if (want_dc) dc = at::empty({c.size(0), c.size(1)}, c.options());
                 if (want_sb) dsb = at::empty({1}, dy.options().dtype(at::kFloat));
-                const int64_t need = rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_KEPT, &d);
-                const Tensor ws = bytes(need, dy);
+                const auto bias = ctx->saved_data["bias"].toIntVector();
+                const BiasGrads g(ctx, dy, bias, has_sb ? 3 : 2);
+                const int64_t least = rdb_linear_workspace_bytes(RDB_OP_LINEAR_BWD_KEPT, &d);
+                if (g.ref.k >= 0) {
+                    const int64_t need = std::max(least, rdb_bias_bwd_workspace_bytes(d.tokens, d.out_f));
+                    const Tensor ws = bytes(need, dy);
+                    check(rdb_linear_bwd_kept_pseudo_bias(ptr(dx), l.in_f, ptr(dc), code(c.scalar_type()), want_sb ? dsb.data_ptr<float>() : nullptr, dy.data_ptr(),
+                                                          dy.stride(0), ptr(xs), want_sb ? xs.stride(0) : l.in_f, kept.data_ptr(), c.data_ptr(), ptr(s), &g.ref, &d,
+                                                          ptr(ws), need, stream_of(dy)),
+                          "rdb_linear_bwd_kept");
+                    if (want_sb) dsb = dsb.to(sb.scalar_type());
+                    db = g.done(bias);
+                    return;
+                }
+                const Tensor ws = bytes(least, dy);
                 check(rdb_linear_bwd_kept(ptr(dx), l.in_f, ptr(dc), code(c.scalar_type()), want_sb ? dsb.data_ptr<float>() : nullptr, dy.data_ptr(), dy.stride(0),
-                                          ptr(xs), want_sb ? xs.stride(0) : l.in_f, kept.data_ptr(), c.data_ptr(), ptr(s), &d, ptr(ws), need, stream_of(dy)),
+                                          ptr(xs), want_sb ? xs.stride(0) : l.in_f, kept.data_ptr(), c.data_ptr(), ptr(s), &d, ptr(ws), least, stream_of(dy)),
                       "rdb_linear_bwd_kept");
                 if (want_sb) dsb = dsb.to(sb.scalar_type());
             }

@@ -66,3 +66,50 @@ def test_many_coefficients():
             best = min(best, start.elapsed_time(end) * 100.0)
         us.append(best)
     assert us[0] < us[1] + 30.0, us
+
+
+# beside the last launch of a layer's backward pass: one tile and many, blocks of 256, 512 and 1024 threads, more outputs than threads, a dy too large for it
+@pytest.mark.parametrize("T,in_f,out_f,k,dtype", [(128, 784, 256, 64, torch.float32), (128, 256, 10, 64, torch.float32), (1, 33, 7, 16, torch.float32), (64, 4100, 1000, 100, torch.float32),
+                                                  (500, 900, 120, 31, torch.float32), (33, 65, 1025, 300, torch.float32), (600, 4000, 100, 16, torch.float32),
+                                                  (300, 200, 300, 64, torch.float32), (129, 301, 77, 50, torch.bfloat16), (300, 3001, 257, 30, torch.bfloat16)])
+@pytest.mark.parametrize("split", [1, 0])
+def test_beside_a_layers_backward_pass(T, in_f, out_f, k, dtype, split):
+    import ctypes
+
+    from randumb_amd import _lib, hip
+
+    print(f"case bias gradient beside {T} tokens {in_f} -> {out_f} k={k} {dtype} split={split}", flush=True)
+    lib, stream, b16 = _lib.load(), torch.cuda.current_stream().cuda_stream, int(dtype == torch.bfloat16)
+    before = hip.set_f32_split(split)
+    try:
+        g = torch.Generator().manual_seed(T + out_f)
+        c, dy = torch.randn(out_f, k, generator=g).to(dtype).cuda(), torch.randn(T, out_f + 3, generator=g).to(dtype).cuda()
+        d = hip._desc(T, in_f, out_f, c, in_f, 1, 5, dtype, 0)
+        ref, kept = ctypes.byref(d), torch.randn(T, k, generator=g).cuda()
+        if not lib.rdb_linear_kept_bytes(ref):
+            pytest.skip("nothing is kept of this layer")
+        room = lib.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_BWD_KEPT, ref)
+        need = max(room, lib.rdb_bias_bwd_workspace_bytes(T, out_f))
+        ws = torch.randint(0, 256, (need + 64,), dtype=torch.uint8, device="cuda")
+        tail = ws[need:].clone()
+        noise, line = hip.sq5_fill_2d(out_f, k, 11).double(), hip.sq5_fill_1d(out_f, 11).double()
+        sums = dy[:, :out_f].double().sum(0)
+        bound = 1.2e-7 * (T * out_f) ** 0.5 * float(dy.double().norm()) + 1e-6   # as above
+        for want_dx, want_dc in ((1, 1), (0, 1), (1, 0), (0, 0)):
+            dx, dc = torch.full((T, in_f), 7.0, device="cuda", dtype=dtype), torch.full((out_f, k), 7.0, device="cuda", dtype=dtype)
+            args = (dx.data_ptr() if want_dx else None, in_f, dc.data_ptr() if want_dc else None, b16, None, dy.data_ptr(), out_f + 3, None, in_f, kept.data_ptr(), c.data_ptr(),
+                    None)
+            assert lib.rdb_linear_bwd_kept(*args, ref, ws.data_ptr(), need, stream) == 0
+            want = dx.clone(), dc.clone()
+            for grads in ((1, 1), (1, 0), (0, 1)):
+                db, ds = torch.full((k + 1,), 7.0, device="cuda"), torch.full((2,), 7.0, device="cuda")
+                dx.fill_(7.0), dc.fill_(7.0)
+                bias = _lib.PseudoBiasGrad(db.data_ptr() if grads[0] else None, ds.data_ptr() if grads[1] else None, k, 11)
+                assert lib.rdb_linear_bwd_kept_pseudo_bias(*args, ctypes.byref(bias), ref, ws.data_ptr(), need, stream) == 0
+                assert torch.equal(dx, want[0]) and torch.equal(dc, want[1])
+                assert float((db[:k].double() - sums @ noise).abs().max()) < bound if grads[0] else bool((db == 7.0).all())
+                assert abs(float(ds[0]) - float(sums @ line)) < bound if grads[1] else float(ds[0]) == 7.0
+                assert float(db[k]) == 7.0 and float(ds[1]) == 7.0 and torch.equal(ws[need:], tail)
+        assert lib.rdb_linear_bwd_kept_pseudo_bias(*args, ctypes.byref(bias), ref, ws.data_ptr(), need - 1, stream) != 0
+    finally:
+        hip.set_f32_split(before)

@@ -408,6 +408,14 @@ int rdb_linear_bwd_projected_rbias(void *dx, int64_t lddx, void *dcoef, int dcoe
                                    const void *scale_bias, const rdb_linear_desc *desc, void *workspace, int64_t workspace_bytes,
                                    void *stream);
 
+/* rdb_linear_bwd_projected_to (dcoef in bf16) of a layer whose input was the squared ReLU of `gate` ([tokens x in_f] bf16, contiguous, as dx is): dx is the
+ * gradient of `gate`, that of the layer's input, in bf16, times 2 relu(gate), in the pass that stores it.  For the layers of which the first call says 1 (bf16, one
+ * chunk of tokens, k <= 256, in_f a multiple of 64); dx 128-byte aligned, gate 16-byte aligned; workspace as rdb_linear_bwd_projected_to. */
+int rdb_linear_bwd_projected_takes_relu_square(const rdb_linear_desc *desc);
+int rdb_linear_bwd_projected_relu_square(void *dx, void *dcoef, const void *dy, int64_t lddy, const void *state, const void *coef,
+                                         const void *gate, const rdb_linear_desc *desc, void *workspace, int64_t workspace_bytes,
+                                         void *stream);
+
 /* The projected form's counterpart for layers without a projection state (bf16 with sizes that are not multiples of 8, fp32
  * in the few-token regime; rdb_linear_kept_bytes says how much, 0: none, use the calls above): the forward pass leaves
  * z = x . N^T (fp32, [tokens x k] row-major) in `kept`, 16-byte aligned, and the backward pass starts from it.  scale_bias as

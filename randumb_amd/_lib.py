@@ -76,6 +76,8 @@ EXPORTS = [
     "rdb_linear_fwd_kept",
     "rdb_linear_fwd_kept_pseudo_bias",
     "rdb_linear_fwd_kept_ws",
+    "rdb_linear_bwd_projected_takes_relu_square",
+    "rdb_linear_bwd_projected_relu_square",
     "rdb_linear_bwd_kept",
     "rdb_linear_bwd_kept_pseudo_bias",
     "rdb_set_big_tiles",
@@ -240,6 +242,10 @@ def load() -> ctypes.CDLL:
     L.rdb_linear_fwd_kept_pseudo_bias.restype = ci
     L.rdb_linear_fwd_kept_ws.argtypes = [vp, i64, vp, vp, i64, vp, vp, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_fwd_kept_ws.restype = ci
+    L.rdb_linear_bwd_projected_takes_relu_square.argtypes = [dp]
+    L.rdb_linear_bwd_projected_takes_relu_square.restype = ci
+    L.rdb_linear_bwd_projected_relu_square.argtypes = [vp, vp, vp, i64, vp, vp, vp, dp, vp, i64, vp]
+    L.rdb_linear_bwd_projected_relu_square.restype = ci
     L.rdb_linear_bwd_kept.argtypes = [vp, i64, vp, ci, vp, vp, i64, vp, i64, vp, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_bwd_kept.restype = ci
     L.rdb_linear_bwd_kept_pseudo_bias.argtypes = [vp, i64, vp, ci, vp, vp, i64, vp, i64, vp, vp, vp, vp, dp, vp, i64, vp]

@@ -11,10 +11,7 @@
 namespace rdb {
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ float lo_f32(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float hi_f32(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
 __device__ __forceinline__ float wave_sum(float v)
 {
@@ -134,12 +131,6 @@ __device__ __forceinline__ uint32_t relu2_pair(uint32_t w)
 {
     const float a = relu(lo_f32(w)), b = relu(hi_f32(w));
     return f32x2_to_bf16x2(a * a, b * b);
-}
-__device__ __forceinline__ uint32_t relu2_grad_pair(uint32_t w, uint32_t d)
-{
-    // 0 where x <= 0 whatever dy is, an infinite or undefined one included
-    const float a = relu(lo_f32(w)), b = relu(hi_f32(w));
-    return f32x2_to_bf16x2(a == 0.0f ? 0.0f : lo_f32(d) * (a + a), b == 0.0f ? 0.0f : hi_f32(d) * (b + b));
 }
 
 template <bool GRAD> __global__ __launch_bounds__(256) void relu_square_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ x,

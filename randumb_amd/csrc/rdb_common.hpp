@@ -123,6 +123,7 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float bf16_to_f32(bf16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
 __device__ __forceinline__ uint32_t f32x2_to_bf16x2(float lo, float hi)
 {
@@ -131,6 +132,15 @@ __device__ __forceinline__ uint32_t f32x2_to_bf16x2(float lo, float hi)
     return __builtin_bit_cast(uint32_t, r);
 }
 __device__ __forceinline__ bf16_t f32_to_bf16(float f) { return (bf16_t)(f32x2_to_bf16x2(f, 0.0f) & 0xffffu); }
+// two bf16 values in a word
+__device__ __forceinline__ float lo_f32(uint32_t w) { return __uint_as_float(w << 16); }
+__device__ __forceinline__ float hi_f32(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
+// the gradient of relu(x)^2, d * 2 relu(x), of two values: 0 where x <= 0 whatever d is, an infinite or undefined one included
+__device__ __forceinline__ uint32_t relu2_grad_pair(uint32_t x, uint32_t d)
+{
+    const float a = lo_f32(x), b = hi_f32(x);
+    return f32x2_to_bf16x2(a <= 0.0f ? 0.0f : lo_f32(d) * (a + a), b <= 0.0f ? 0.0f : hi_f32(d) * (b + b));
+}
 
 template <typename T> struct elem;
 template <> struct elem<float> {

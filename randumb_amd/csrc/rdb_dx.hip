@@ -312,11 +312,11 @@ struct BwdBsParams {
     int tn_blocks;
 };
 
-template <int KG, int AUX, bool TABLE> __global__ __launch_bounds__(ST_THREADS, 1) void bwd_tns_red_kernel(BwdBsParams p)
+template <int KG, int AUX, bool TABLE, bool GATE = false> __global__ __launch_bounds__(ST_THREADS, 1) void bwd_tns_red_kernel(BwdBsParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     if ((int)blockIdx.x < p.tn_blocks)
-        stationary_block<KG, false, !TABLE, AUX, true, TABLE>(p.tn, smem_raw, blockIdx.x);
+        stationary_block<KG, false, !TABLE, AUX, true, TABLE, GATE>(p.tn, smem_raw, blockIdx.x);
     else
         red_block(p.red, blockIdx.x - p.tn_blocks, gridDim.x - p.tn_blocks);
 }
@@ -467,6 +467,12 @@ int linear_dx_factored(void *dx, int64_t lddx, const void *dy, int64_t lddy, con
     return launch_engine(dx_tn_kernel, p2, items, engine_smem<K2_BI, K2_BT, X_BK, K_CONT, K_CONT>(), s, "dx_tn_kernel");
 }
 
+// Whether dx may leave through the gradient of a squared ReLU: where t stays in registers and rows are whole lines (the other kernels are not built for it)
+bool linear_bwd_projected_gates(const rdb_linear_desc *d, const void *dx, int64_t lddx, const void *gate)
+{
+    return dx_factored_ok(d) && tn_stationary_ok(d, lddx) && lddx % 64 == 0 && ((uintptr_t)dx & 127) == 0 && ((uintptr_t)gate & 15) == 0;
+}
+
 // Which of the two launches linear_bwd_projected enqueues: bit 0 the first, bit 1 the second (3: both).  Timing tools launch one
 // of them alone (rdb_linear_bwd_projected_part); the mask is the calling thread's.
 static thread_local int g_bwd_parts = 3;
@@ -485,11 +491,14 @@ static int table_blocks(uint32_t pieces, int num_cus) { return (int)std::min<int
 // dc_bf16: dcoef is bf16 [out_f x k], the fp32 sums rounded once by the blocks that add them up (needs the workspace with room
 // for the sums, linear_bwd_projected_workspace(d, num_cus, true), and is not combined with accumulate).
 // rb: NULL, or the fused random bias's share, for layers whose t stays in registers otherwise (tn_stationary_ok).
+// gate: NULL, or a matrix as dx is: dx = (dy.C).N * 2 relu(gate), where linear_bwd_projected_gates.
 int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, int64_t lddy, const void *z, const void *coef,
                          const rdb_linear_desc *d, int num_cus, void *workspace, int64_t workspace_bytes, bool accumulate, bool dc_bf16,
-                         hipStream_t s, const RBiasDx *rb)
+                         hipStream_t s, const RBiasDx *rb, const void *gate)
 {
     if (!dx_factored_ok(d)) return RDB_E_UNSUPPORTED;
+    if (gate && (rb || accumulate || !linear_bwd_projected_gates(d, dx, lddx, gate) || workspace_bytes < linear_bwd_projected_workspace(d, num_cus, dc_bf16)))
+        return RDB_E_UNSUPPORTED;
     if (rb && (accumulate || !tn_stationary_ok(d, lddx) || workspace_bytes < linear_bwd_projected_workspace(d, num_cus, dc_bf16))) return RDB_E_UNSUPPORTED;
     if (dc_bf16 && (accumulate || workspace_bytes < linear_bwd_projected_workspace(d, num_cus, true))) return RDB_E_UNSUPPORTED;
     if (!workspace || workspace_bytes < linear_dx_factored_workspace(d) || ((uintptr_t)workspace & 15)) return RDB_E_UNSUPPORTED;
@@ -584,9 +593,12 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             if (rblocks < 1) rblocks = 1;
             if (direct) rblocks = 0;
             bs.tn.coef = n;
+            bs.tn.gate = static_cast<const bf16_t *>(gate);
             return with_stationary_variant(bs.tn, [&](auto kg, auto aux) {
                 constexpr int KG = decltype(kg)::value, AUX = decltype(aux)::value;
                 auto kernel = n ? bwd_tns_red_kernel<KG, AUX, (KG > 2)> : bwd_tns_red_kernel<KG, AUX, false>;   // no table up to k = 128
+                if constexpr (AUX == Y_STREAM)
+                    if (gate) kernel = n ? bwd_tns_red_kernel<KG, AUX, (KG > 2), true> : bwd_tns_red_kernel<KG, AUX, false, true>;
                 const size_t smem_s = stationary_smem(kg);
                 if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem_s, "bwd_tns_red_kernel")) return rl;
                 kernel<<<bs.tn_blocks + rblocks, ST_THREADS, smem_s, s>>>(bs);

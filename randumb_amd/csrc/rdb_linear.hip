@@ -339,7 +339,8 @@ int linear_dcoef_f32(float *dcoef, float *d_scale_bias, const void *dy, int64_t 
 // rdb_dx.hip
 int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, int64_t lddy, const void *z, const void *coef,
                          const rdb_linear_desc *d, int num_cus, void *workspace, int64_t workspace_bytes, bool accumulate, bool dc_bf16,
-                         hipStream_t s, const RBiasDx *rb = nullptr);
+                         hipStream_t s, const RBiasDx *rb = nullptr, const void *gate = nullptr);
+bool linear_bwd_projected_gates(const rdb_linear_desc *d, const void *dx, int64_t lddx, const void *gate);
 int64_t linear_dx_factored_workspace(const rdb_linear_desc *d);
 int64_t linear_bwd_projected_workspace(const rdb_linear_desc *d, int num_cus, bool force_partial);
 int linear_dx_factored(void *dx, int64_t lddx, const void *dy, int64_t lddy, const void *coef, const void *scale_bias,
@@ -1273,7 +1274,7 @@ static int64_t bwd_projected_workspace(const rdb_linear_desc *d, bool force_part
 static int64_t bwd_projected_extra(const rdb_linear_desc *d) { return chunk_plan(d).nchunks == 1 ? linear_bwd_projected_extra(d, num_compute_units()) : 0; }
 
 static int bwd_projected_entry(const char *who, void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, const void *dy, int64_t lddy, const void *z,
-                               const void *coef, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
+                               const void *coef, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream, const void *gate = nullptr)
 {
     if (f32_projected(d)) {   // dx may be NULL: the coefficient gradient alone
         if (int rc = check_projected_f32(who, d)) return rc;
@@ -1307,7 +1308,7 @@ static int bwd_projected_entry(const char *who, void *dx, int64_t lddx, void *dc
         const rdb_linear_desc dd = chunk_desc(d, pl, c);
         rc = linear_bwd_projected(at_bytes(dx, c * pl.chunk_tokens * lddx * 2), lddx, static_cast<float *>(dcoef),
                                   at_bytes(dy, c * pl.chunk_tokens * lddy * 2), lddy, at_bytes(z, c * pl.state_stride), coef, &dd,
-                                  num_compute_units(), workspace, workspace_bytes, c > 0, dc_bf16, (hipStream_t)stream);
+                                  num_compute_units(), workspace, workspace_bytes, c > 0, dc_bf16, (hipStream_t)stream, nullptr, gate);
         if (rc == RDB_E_UNSUPPORTED) return set_error(RDB_E_UNSUPPORTED, "%s: internal: chunk %d of %d refused", who, c, pl.nchunks);
         if (rc) return rc;
     }
@@ -1389,6 +1390,25 @@ extern "C" int rdb_linear_bwd_projected_to(void *dx, int64_t lddx, void *dcoef, 
                                            const void *coef, const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
 {
     return bwd_projected_entry("rdb_linear_bwd_projected_to", dx, lddx, dcoef, dcoef_dtype, dy, lddy, z, coef, d, workspace, workspace_bytes, stream);
+}
+
+// One chunk of tokens, and a kernel that applies the gate as it stores dx
+static bool takes_relu_square(const rdb_linear_desc *d, const void *dx, const void *gate)
+{
+    ChunkPlan pl;
+    return !f32_projected(d) && d->coef_dtype == RDB_BF16 && !check_projected("rdb_linear_bwd_projected_takes_relu_square", d, &pl) && pl.nchunks == 1 &&
+           linear_bwd_projected_gates(d, dx, d->in_f, gate);
+}
+extern "C" int rdb_linear_bwd_projected_takes_relu_square(const rdb_linear_desc *d) { return d && takes_relu_square(d, nullptr, nullptr) ? 1 : 0; }
+
+extern "C" int rdb_linear_bwd_projected_relu_square(void *dx, void *dcoef, const void *dy, int64_t lddy, const void *z, const void *coef, const void *gate,
+                                                    const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
+{
+    const char *who = "rdb_linear_bwd_projected_relu_square";
+    if (!d || !gate) return set_error(RDB_E_NULL, "%s: desc or gate is NULL", who);
+    if (!takes_relu_square(d, dx, gate))
+        return set_error(RDB_E_UNSUPPORTED, "%s: layers of which rdb_linear_bwd_projected_takes_relu_square says so; dx 128-byte aligned, gate 16-byte aligned", who);
+    return bwd_projected_entry(who, dx, d->in_f, dcoef, RDB_BF16, dy, lddy, z, coef, d, workspace, workspace_bytes, stream, gate);
 }
 
 // ----------------------------------------------------------------------------------------------- z kept from forward to backward

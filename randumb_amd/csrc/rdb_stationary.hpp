@@ -32,6 +32,7 @@ struct StParams {
     const bf16_t *coef;  // right operand [out_f x k], or (TABLE) in fragment order; not used when the right operand is noise
     const bf16_t *bias;  // [out_f] or NULL
     bf16_t *y;           // [tokens x out_f], leading dimension ldy
+    const bf16_t *gate;  // GATE: as y is
     int64_t ldy;
     int tokens, out_f, k;
     int tiles_t, splits, units_per_split;
@@ -49,19 +50,23 @@ struct StParams {
 // (exact in bf16).  AUX: cache policy of the row stores (an immediate of the instruction: two copies of the steps in one kernel cost it 10 to 20
 // registers, and spills with k = 256 and a bias).
 // TABLE: `coef` is in fragment order (rows padded to 32, k to kpad, zeros there): a unit's tile is consecutive kilobytes.
-template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE> struct StBlock {
+// GATE: the rows leave as y * 2 relu(gate) (relu2_grad_pair of their bf16 values), the input gradient of a layer behind a squared ReLU: the product's
+// rows are not written, read again and written.  A unit's pieces of gate are loaded in its own step and used a step later, behind a unit's matrix
+// instructions, which also cover the arithmetic (200 vector instructions a wave and unit beside 32 matrix instructions).
+template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE, bool GATE> struct StBlock {
     static constexpr int kpad = KG * 64, ldk = kpad + 8, cpr = kpad / 8, ncp = ST_BO * cpr, NQ = ncp / ST_THREADS;
     const StParams &p;
     bf16_t *Cs;   // [2][64 rows][ldk]
     bf16_t *stg;  // this wave's [32 tok][72]
     int lane, r, g, unit0, nunits;
-    __amdgpu_buffer_rsrc_t rs_c, rs_y, rs_b;
+    __amdgpu_buffer_rsrc_t rs_c, rs_y, rs_b, rs_g;
     f32x4 rc[NQ];
     int t;
     bf16x8 zf[KG * 4];
     uint2 braw[2][4];   // bias of the unit whose epilogue comes next: four output features per (mi, jq) of this lane
     int tok_y;          // token of the row piece this lane stores in step 0 of the epilogue; step q: 8 q further
     uint32_t off_y;     // its byte offset in y at output feature 0
+    u32x4 graw[GATE ? 4 : 1];   // gate of the unit whose epilogue comes next, as the row pieces of y
 
     __device__ __forceinline__ void issue(int unit)
     {   // global -> registers for a C tile; rows past out_f read as zeros
@@ -137,6 +142,17 @@ template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE> struct StBlock {
                     braw[mi][jq] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rs_b, o < p.out_f ? o * 2 : (int)BUFFER_OOB, 0, 0));
                 }
             }
+        auto piece = [&](int at, int qq) {   // byte offset in y of this lane's row piece qq of the unit at output feature `at`
+            return at + (lane & 7) * 8 < p.out_f && tok_y + qq * 8 < p.tokens ? off_y + (uint32_t)(qq * 8 * (int)p.ldy * 2 + at * 2) : BUFFER_OOB;
+        };
+        u32x4 gnow[4];
+        if constexpr (GATE) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                gnow[q] = graw[q];
+                if (MMA) graw[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_g, (int)piece(o0 + ST_BO, q), 0, 0));
+            }
+        }
         // the epilogue in 10 small operations, so that few values are in flight at a time: 8 x (accumulators of 8 output features
         // -> + bias -> bf16 -> patch[tok][o]), then 2 x (16 tokens: rows of 128 bytes out of the patch)
         auto epilogue_op = [&](int op) {
@@ -160,8 +176,13 @@ template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE> struct StBlock {
 #pragma unroll
                 for (int q = 0; q < 2; ++q) {
                     const int qq = h * 2 + q;
-                    const uint32_t a = (o0 + (lane & 7) * 8 < p.out_f && tok_y + qq * 8 < p.tokens)
-                                           ? off_y + (uint32_t)(qq * 8 * (int)p.ldy * 2 + o0 * 2) : BUFFER_OOB;
+                    if constexpr (GATE) {
+                        u32x4 d = __builtin_bit_cast(u32x4, v[q]);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) d[i] = relu2_grad_pair(gnow[qq][i], d[i]);
+                        v[q] = __builtin_bit_cast(f32x4, d);
+                    }
+                    const uint32_t a = piece(o0, qq);
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v[q]), rs_y, (int)a, 0, AUX);
                 }
                 if (op == 9) __builtin_amdgcn_wave_barrier();
@@ -213,10 +234,10 @@ template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE> struct StBlock {
 };
 
 // `block`: index of this block among the blocks that run this body; all ST_THREADS threads of the block must call.
-template <int KG, bool BIAS, bool NOISE, int AUX, bool ZFRAG = false, bool TABLE = false>
+template <int KG, bool BIAS, bool NOISE, int AUX, bool ZFRAG = false, bool TABLE = false, bool GATE = false>
 __device__ __forceinline__ void stationary_block(const StParams &p, unsigned char *smem_raw, int block)
 {
-    typedef StBlock<KG, BIAS, NOISE, AUX, TABLE> B;
+    typedef StBlock<KG, BIAS, NOISE, AUX, TABLE, GATE> B;
     const int t = threadIdx.x, wave = t >> 6;
     // work item = (token tile, split), split fastest: neighbours share the left operand's tile, everyone shares the right operand
     const int w = xcd_work_item(block, p.tiles_t * p.splits);
@@ -236,6 +257,7 @@ __device__ __forceinline__ void stationary_block(const StParams &p, unsigned cha
                                                NOISE ? 0 : TABLE ? (p.out_f + 31) / 32 * 32 * B::kpad * 2 : (int)((int64_t)p.out_f * p.k * 2), 0x00020000);
     b.rs_y = __builtin_amdgcn_make_buffer_rsrc(p.y, 0, (int)(((int64_t)(p.tokens - 1) * p.ldy + p.out_f) * 2), 0x00020000);
     b.rs_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(p.bias), 0, p.bias ? p.out_f * 2 : 0, 0x00020000);  // no bias: zeros
+    if constexpr (GATE) b.rs_g = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(p.gate), 0, (int)(((int64_t)(p.tokens - 1) * p.ldy + p.out_f) * 2), 0x00020000);
     b.t = t;
     if constexpr (ZFRAG) {
         // the fragments lie ready in memory, a k-step of a wave's 32 tokens in 1024 consecutive bytes: no staging, no barrier
@@ -357,6 +379,7 @@ inline int make_stationary_grid(StParams &q, int64_t tokens, int64_t out_f, int 
 {
     q.tokens = (int)tokens;
     q.out_f = (int)out_f;
+    q.gate = nullptr;
     q.sync = nullptr;   // the left operand comes from an earlier launch unless the caller says otherwise afterwards
     q.sync_tag = 0;
     q.sync_n = 0;

@@ -497,16 +497,21 @@ class OneCallLinear : public Function<OneCallLinear> {
 };
 
 // ----------------------------------------------------------------------------------------------- projected form
+Tensor dense(const Tensor &t);
+Tensor relu_squared(const Tensor &x, const Tensor &dy = Tensor());   // relu(x)^2, or with dy its gradient
+Tensor relu_squared_with_graph(const Tensor &x, const Tensor &dy);
 // The forward pass keeps z = x.N^T (and, in bf16, the transposed coefficients) for the backward pass, which needs nothing else
 // of x; with the fused random bias its full-rank share is added on top in both directions and x is saved as well.
+// squared: the layer's input is relu(x)^2, which nothing keeps, and its gradient goes through that on its way to memory (8192 tokens x 3072 -> 768, k = 256:
+// backward and a pass over its dx 62.8 us, 47.7 so).
 class ProjectedLinear : public Function<ProjectedLinear> {
   public:
     static Tensor forward(AutogradContext *ctx, const Tensor &x0, const Tensor &coefs, const OptTensor &bias, const OptTensor &bias_scale, int64_t bias_seed,
-                          const OptTensor &scale_bias, const Layer &l)
+                          const OptTensor &scale_bias, const Layer &l, bool squared)
     {
         const Bias pb{bias, bias_scale, bias_seed};
-        const Tensor x = near_act(x0), c = coefs.contiguous();
-        const c10::OptionalDeviceGuard guard(x.device());
+        const c10::OptionalDeviceGuard guard(x0.device());
+        const Tensor x = squared ? relu_squared(x0) : near_act(x0), c = coefs.contiguous();
         const rdb_linear_desc d = desc(x, l, c);
         const int64_t need = rdb_linear_projection_bytes(&d);
         Tensor state = bytes(need, x), y = at::empty({x.size(0), l.out_f}, x.options());
@@ -532,8 +537,8 @@ class ProjectedLinear : public Function<ProjectedLinear> {
             check(rdb_linear_rbias_fwd_ws(y.data_ptr(), l.out_f, x.data_ptr(), x.stride(0), sb.data_ptr(), &r, ptr(ws), room, s), "rdb_linear_rbias_fwd");
         }
         tick(x);
-        ctx->save_for_backward({state, coefs, scale_bias.value_or(Tensor()), scale_bias ? x0 : Tensor()});
-        ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, (int64_t)l.seed, scale_bias ? 1 : 0, pb.tensors(), coefs.size(1)};
+        ctx->save_for_backward({state, coefs, scale_bias.value_or(Tensor()), scale_bias || squared ? x0 : Tensor()});
+        ctx->saved_data["layer"] = std::vector<int64_t>{l.in_f, l.out_f, (int64_t)l.seed, scale_bias ? 1 : 0, pb.tensors(), coefs.size(1), squared ? 1 : 0};
         ctx->saved_data["bias"] = pb.meta();
         return y;
     }
@@ -541,12 +546,15 @@ class ProjectedLinear : public Function<ProjectedLinear> {
     {
         Tensor dx, dc, ds;
         std::pair<Tensor, Tensor> db;
-        gradients(ctx, grads, dx, dc, ds, db);
         const auto m = ctx->saved_data["layer"].toIntVector();
+        const bool graph = at::GradMode::is_enabled();   // relu(x)^2 is then gone through by stock operators, which have further derivatives
+        gradients(ctx, grads, dx, dc, ds, db, m[6] && !graph);
         layer_gradients(grads[0], m[3] ? (int)(2 + m[4]) : -1, dx, dc, ds, db, ctx->saved_data["bias"].toIntVector());
-        return {dx, dc, db.first, db.second, Tensor(), ds, Tensor()};
+        if (m[6] && graph && dx.defined()) dx = relu_squared_with_graph(ctx->get_saved_variables()[3], dx);
+        return {dx, dc, db.first, db.second, Tensor(), ds, Tensor(), Tensor()};
     }
-    static void gradients(AutogradContext *ctx, const variable_list &grads, Tensor &dx, Tensor &dc, Tensor &dsb, std::pair<Tensor, Tensor> &db)
+    // through: dx is to be the gradient behind relu(x)^2
+    static void gradients(AutogradContext *ctx, const variable_list &grads, Tensor &dx, Tensor &dc, Tensor &dsb, std::pair<Tensor, Tensor> &db, bool through)
     {
         const auto saved = ctx->get_saved_variables();
         const Tensor &state = saved[0], &coefs = saved[1], &scale_bias = saved[2];
@@ -555,11 +563,12 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         const bool has_sb = m[3] != 0;
         constexpr const char *who = "linear (backward)";
         restored(who, coefs, grads[0], {l.out_f, m[5]});
-        if (has_sb) {
-            restored(who, scale_bias, grads[0], scale_bias.sizes());
-            restored(who, saved[3], grads[0], {grads[0].size(0), l.in_f});
-        }
+        if (has_sb) restored(who, scale_bias, grads[0], scale_bias.sizes());
+        if (has_sb || m[6]) restored(who, saved[3], grads[0], {grads[0].size(0), l.in_f});
         const at::AutoGradMode no_grad(false);
+        through = through && ctx->needs_input_grad(0);
+        const Tensor gate = through ? dense(saved[3]) : Tensor();
+        if (through) restored_values(who, gate, grads[0], at::kBFloat16, grads[0].size(0) * l.in_f);
         const bool want_x = ctx->needs_input_grad(0), want_dc = ctx->needs_input_grad(1), want_sb = has_sb && ctx->needs_input_grad(2 + m[4]);
         const bool want_dx = want_x || want_sb;   // the gradient of the scale comes out of the random-bias share of dx
         Tensor dy = near_act(grads[0]);
@@ -590,11 +599,18 @@ class ProjectedLinear : public Function<ProjectedLinear> {
             const Tensor ws = bytes(need, dy);
             if (want_dx) dx = at::empty({dy.size(0), l.in_f}, dy.options());
             dc = at::empty({c.size(0), c.size(1)}, dy.options().dtype(to_bf16 ? at::kBFloat16 : at::kFloat));
-            check(to_bf16 ? rdb_linear_bwd_projected_to(ptr(dx), l.in_f, dc.data_ptr(), RDB_BF16, dy.data_ptr(), dy.stride(0), state.data_ptr(), c.data_ptr(),
-                                                        &d, ptr(ws), need, s)
-                          : rdb_linear_bwd_projected(ptr(dx), l.in_f, dc.data_ptr<float>(), dy.data_ptr(), dy.stride(0), state.data_ptr(), c.data_ptr(), &d,
-                                                     ptr(ws), need, s),
-                  "rdb_linear_bwd_projected");
+            if (through && to_bf16 && rdb_linear_bwd_projected_takes_relu_square(&d) && (uintptr_t)dx.data_ptr() % 128 == 0) {
+                check(rdb_linear_bwd_projected_relu_square(dx.data_ptr(), dc.data_ptr(), dy.data_ptr(), dy.stride(0), state.data_ptr(), c.data_ptr(), gate.data_ptr(), &d,
+                                                           ptr(ws), need, s),
+                      "rdb_linear_bwd_projected_relu_square");
+                through = false;
+            } else {
+                check(to_bf16 ? rdb_linear_bwd_projected_to(ptr(dx), l.in_f, dc.data_ptr(), RDB_BF16, dy.data_ptr(), dy.stride(0), state.data_ptr(), c.data_ptr(),
+                                                            &d, ptr(ws), need, s)
+                              : rdb_linear_bwd_projected(ptr(dx), l.in_f, dc.data_ptr<float>(), dy.data_ptr(), dy.stride(0), state.data_ptr(), c.data_ptr(), &d,
+                                                         ptr(ws), need, s),
+                      "rdb_linear_bwd_projected");
+            }
             dc = dc.to(c.scalar_type());
         } else if (want_dx) {
             dx = linear_bwd_dx(dy, c, l, Tensor());
@@ -621,6 +637,7 @@ class ProjectedLinear : public Function<ProjectedLinear> {
             }
         }
         if (!want_x) dx = Tensor();
+        if (through && dx.defined()) dx = relu_squared(gate, dx);
         db = bias_grads(ctx, dy, ctx->saved_data["bias"].toIntVector(), 2);
     }
 };
@@ -957,30 +974,34 @@ class AddRmsNorm : public Function<AddRmsNorm> {
     }
 };
 
+Tensor relu_squared(const Tensor &x0, const Tensor &dy0)
+{
+    const Tensor x = dense(x0), dy = dy0.defined() ? dense(dy0) : Tensor();
+    const c10::OptionalDeviceGuard guard(x.device());
+    Tensor out = at::empty_like(x);
+    check(rdb_relu_square(out.data_ptr(), x.data_ptr(), ptr(dy), x.numel(), stream_of(x)), "rdb_relu_square");
+    return out;
+}
+Tensor relu_squared_with_graph(const Tensor &x, const Tensor &dy)
+{
+    return stock_gradient([](const variable_list &in) { return variable_list{at::relu(in[0]).square()}; }, {x}, {dy})[0];
+}
 class ReluSquare : public Function<ReluSquare> {
   public:
     static Tensor forward(AutogradContext *ctx, const Tensor &x0)
     {
-        const Tensor x = dense(x0);
-        const c10::OptionalDeviceGuard guard(x.device());
-        Tensor y = at::empty_like(x);
-        check(rdb_relu_square(y.data_ptr(), x.data_ptr(), nullptr, x.numel(), stream_of(x)), "rdb_relu_square");
         ctx->save_for_backward({x0});
-        return y;
+        return relu_squared(x0);
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads)
     {
         const Tensor x0 = ctx->get_saved_variables()[0];
         constexpr const char *who = "relu_square (backward)";
         restored(who, x0, grads[0], grads[0].sizes());
-        if (at::GradMode::is_enabled())
-            return stock_gradient([](const variable_list &in) { return variable_list{at::relu(in[0]).square()}; }, {x0}, {grads[0]});
+        if (at::GradMode::is_enabled()) return {relu_squared_with_graph(x0, grads[0])};
         const Tensor x = dense(x0), dy = dense(grads[0]);
         restored_values(who, x, dy, at::kBFloat16, dy.numel());
-        const c10::OptionalDeviceGuard guard(x.device());
-        Tensor dx = at::empty_like(x);
-        check(rdb_relu_square(dx.data_ptr(), x.data_ptr(), dy.data_ptr(), x.numel(), stream_of(x)), "rdb_relu_square");
-        return {dx};
+        return {relu_squared(x, dy)};
     }
 };
 
@@ -1180,7 +1201,23 @@ PyObject *py_linear_projected(PyObject *, PyObject *const *a, Py_ssize_t n)
         // without a backward pass to come there is no state to keep: the one-call forward
         if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
             return THPVariable_Wrap(linear_fwd(x, c, l, sb, b));
-        return THPVariable_Wrap(ProjectedLinear::apply(x, c, b.coef, b.scale, b.seed, sb, l));
+        return THPVariable_Wrap(ProjectedLinear::apply(x, c, b.coef, b.scale, b.seed, sb, l, false));
+    });
+}
+
+// relu_square_linear(x, coefs, in_f, out_f, seed): linear_projected of relu(x)^2, for a backward pass to come (None without one, or where
+// ops.linear runs another form)
+PyObject *py_relu_square_linear(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 5);
+        const Tensor &x = tensor_arg(a[0]), &c = tensor_arg(a[1]);
+        const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[2]), 1, seed_arg(a[4])};
+        same_device("linear_fwd", x, {&c});
+        check_sizes("linear_fwd", x, c, l, OptTensor(), Bias{});
+        if (!past_dispatcher({&x, &c}) || !at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad())) Py_RETURN_NONE;
+        need_bf16("relu_square_linear", x);
+        return THPVariable_Wrap(ProjectedLinear::apply(x, c, OptTensor(), OptTensor(), -1, OptTensor(), l, true));
     });
 }
 
@@ -1334,7 +1371,7 @@ PyObject *py_set_hooks(PyObject *, PyObject *const *a, Py_ssize_t n)
 }
 
 #define RDB_METHOD(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {RDB_METHOD(takes_projected),   RDB_METHOD(linear_projected), RDB_METHOD(linear_one_call),
+PyMethodDef methods[] = {RDB_METHOD(takes_projected),   RDB_METHOD(linear_projected), RDB_METHOD(linear_one_call), RDB_METHOD(relu_square_linear),
                          RDB_METHOD(linear_vector),     RDB_METHOD(embed_rows),       RDB_METHOD(set_hooks),
                          RDB_METHOD(rms_norm),          RDB_METHOD(add_rms_norm),     RDB_METHOD(relu_square),
                          RDB_METHOD(cross_entropy),     RDB_METHOD(causal_attention), RDB_METHOD(once_differentiable),

@@ -18,7 +18,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from . import _lib
+from . import _lib, ops
 from .SillyLayers import SillyEmbedding, SillyLinear
 
 
@@ -119,6 +119,12 @@ class RT_CausalSelfAttention(nn.Module):
         return self.c_proj(y.transpose(1, 2).reshape(B, T, D))
 
 
+def _unhooked(m: nn.Module) -> bool:
+    """Nothing that has to see ``m`` called: no replaced method, no compiled call, no hooks."""
+    return ("forward" not in m.__dict__ and type(m).__call__ is _MODULE_CALL and m._compiled_call_impl is None and not torch.nn.modules.module._has_any_global_hook()
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks))
+
+
 class RT_MLP(nn.Module):
     def __init__(self, dim: int, config: RT_GPTConfig):
         super().__init__()
@@ -128,8 +134,28 @@ class RT_MLP(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         h = self.c_fc(x)
         ext = _fused(h)
-        a = None if ext is None else ext.relu_square(h)
+        if ext is None:
+            return self.c_proj(F.relu(h).square())
+        y = self._proj_of_relu_square(h, ext)
+        if y is not None:
+            return y
+        a = ext.relu_square(h)
         return self.c_proj(F.relu(h).square() if a is None else a)
+
+    def _proj_of_relu_square(self, h: torch.Tensor, ext):
+        """Both in one autograd node, whose backward pass needs no pass over memory of its own for the activation; None where the layer is
+        more than its forward, or no backward pass is to come."""
+        p = self.c_proj
+        if not (torch.is_grad_enabled() and type(p) is RT_CastedLinear and RT_CastedLinear.forward is _LINEAR_FORWARD and _unhooked(p)):
+            return None
+        w, coef, in_f, out_f = p._buffers.get("weight"), p._parameters.get("weight_coef"), p.in_features, p.out_features
+        if w is None or coef is None or w.fused_bias or p.bias is not None or not p.fused or h.dtype != w.dtype or h.shape[-1] != in_f or ops._tracing():
+            return None
+        x = h.reshape(-1, in_f)
+        if not ext.takes_projected(x, coef, in_f, out_f, in_f, 1, None, None):
+            return None
+        y = ext.relu_square_linear(x, coef, in_f, out_f, w.seed)
+        return None if y is None else y.reshape(*h.shape[:-1], out_f)
 
 
 class RT_Block(nn.Module):
@@ -150,12 +176,11 @@ class RT_Block(nn.Module):
 
     def _plain(self) -> bool:
         """Nothing that has to see ``forward`` run: no subclass, no replaced method, no compiled call, no hooks."""
-        return (type(self) is RT_Block and "forward" not in self.__dict__ and RT_Block.forward is _BLOCK_FORWARD and RT_Block.__call__ is _MODULE_CALL
-                and self._compiled_call_impl is None and not torch.nn.modules.module._has_any_global_hook()
-                and not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks or self._backward_pre_hooks))
+        return type(self) is RT_Block and RT_Block.forward is _BLOCK_FORWARD and _unhooked(self)
 
 
-_BLOCK_FORWARD, _MODULE_CALL = RT_Block.forward, nn.Module.__call__   # as they stand here: replaced ones are called
+# as they stand here: replaced ones are called
+_BLOCK_FORWARD, _LINEAR_FORWARD, _MODULE_CALL = RT_Block.forward, RT_CastedLinear.forward, nn.Module.__call__
 
 
 class RT_GPT(nn.Module):

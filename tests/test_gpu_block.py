@@ -303,3 +303,49 @@ def test_the_fused_model_is_no_further_from_64_bits_than_the_stock_one(ext, monk
     # One number, so chance alone decides which loss is nearer.  A logit (0.3 typically) is off by some 1.4e-2 of itself, as the gradients
     # are; over 576 rows the mean is off by 4e-3 / 24 = 1.8e-4, 2.5e-5 of a loss of 6.9.  Four times that.
     assert off[True]["loss"] <= 1e-4 and off[False]["loss"] <= 1e-4
+
+
+@pytest.mark.parametrize("dim,k,tokens", [(64, 64, 40), (192, 136, 700), (128, 264, 300), (72, 64, 520)])
+@pytest.mark.parametrize("kind", ["all", "frozen coefficients", "frozen input", "saved elsewhere", "second derivative"])
+def test_squared_relu_in_the_projections_node(dim, k, tokens, kind):
+    """The activation in c_proj's autograd node against a c_proj with a hook, which is called for itself: bit for bit, also where dx is not stored through
+    the activation's gradient (k > 256, features that are no whole lines)."""
+    from randumb_amd.gpt import RT_GPTConfig, RT_MLP
+
+    print(f"case squared ReLU in the projection's node dim={dim} k={k} {kind}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(dim)
+    with torch.device("cuda"):
+        mlp = RT_MLP(dim, RT_GPTConfig(int_dim_gen=iter([k, k]), seed_gen=iter([3, 4]))).bfloat16()
+    with torch.no_grad():
+        for m in (mlp.c_fc, mlp.c_proj):
+            m.weight_coef.normal_(0.0, (3.0 / k) ** 0.5, generator=g)
+    x, dy = bf16(g, 2, tokens // 2, dim).requires_grad_(), bf16(g, 2, tokens // 2, dim)
+    leaves = [x, mlp.c_fc.weight_coef, mlp.c_proj.weight_coef]
+    if kind == "frozen coefficients":
+        leaves.pop().requires_grad_(False)
+    if kind == "frozen input":
+        x.requires_grad_(False), mlp.c_fc.weight_coef.requires_grad_(False)
+        leaves = leaves[2:]
+
+    def run():
+        if kind == "saved elsewhere":
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.cuda()):
+                y = mlp(x)
+        else:
+            y = mlp(x)
+        if kind == "second derivative":   # of c_proj's input gradient behind the activation, in what feeds the activation
+            first = torch.autograd.grad(y, leaves, dy, create_graph=True)
+            with pytest.raises(RuntimeError, match="no second derivative"):
+                torch.autograd.grad(first[2].float().sum(), leaves[2], retain_graph=True, allow_unused=True)
+                torch.autograd.grad(first[0].float().square().sum(), x)
+            return y, [f.detach() for f in first]
+        return y, torch.autograd.grad(y, leaves, dy)
+
+    y, grads = run()
+    assert "Projected" in y.grad_fn.name() or "Projected" in y.grad_fn.next_functions[0][0].name()
+    seen = []
+    mlp.c_proj.register_forward_hook(lambda m, args, out: seen.append(args[0]))
+    y2, grads2 = run()
+    assert len(seen) == 1 and torch.equal(y, y2) and all(torch.equal(a, b) for a, b in zip(grads, grads2))
+    node = lambda t: t.grad_fn.next_functions[0][0].next_functions[0][0]
+    assert not torch.is_grad_enabled() or kind == "frozen input" or "ReluSquare" not in str(node(y)) and "ReluSquare" in str([node(y2)] + [f[0] for f in node(y2).next_functions])

@@ -39,3 +39,50 @@ def test_from_memory_is_hashed_in_place(T, in_f, out_f, k):
         assert torch.equal(dx, results[0][0]) and torch.equal(dc.bfloat16(), results[0][1])
     want = dy[:, :out_f].double() @ C.double() @ hip.sq5_fill_2d(in_f, k, 9).double().t()
     assert float((results[0][0].double() - want).norm() / want.norm()) < 6e-3   # N, t and dx rounded to bf16 once each, 1.13e-3 as a norm; 2^-9 at most
+
+
+# t in one to four groups of 64 coefficients, N hashed and from memory, the last tiles of tokens and features not full
+@pytest.mark.parametrize("T,in_f,out_f,k", [(1, 64, 8, 8), (255, 64, 40, 64), (300, 192, 136, 72), (257, 320, 64, 128), (700, 960, 256, 136), (3300, 3072, 768, 192),
+                                            (3333, 2048, 512, 256), (1000, 4096, 264, 250 // 8 * 8)])
+def test_dx_through_the_gradient_of_a_squared_relu(T, in_f, out_f, k):
+    """Bit for bit what the backward call and the pass over its dx give, infinities and NaNs included."""
+    import ctypes
+
+    from randumb_amd import _lib, hip
+
+    print(f"case dx through a squared ReLU T={T} {in_f} -> {out_f} k={k}", flush=True)
+    lib, stream, bf = _lib.load(), torch.cuda.current_stream().cuda_stream, torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(T + k)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").to(bf)
+    h, c, dy = rand(T, in_f), rand(out_f, k), rand(T, out_f)
+    h.view(-1)[::97], h.view(-1)[5::101], h.view(-1)[7::103], h.view(-1)[9::107] = 0.0, float("inf"), float("nan"), -float("inf")
+    dy[T // 2, 0] = float("inf")
+    y, state = hip.linear_project_fwd(rand(T, in_f), c, 5, None)
+    d = hip._desc(T, in_f, out_f, c, in_f, 1, 5, bf, 0)
+    ref = ctypes.byref(d)
+    assert lib.rdb_linear_bwd_projected_takes_relu_square(ref) == 1
+    need = lib.rdb_linear_workspace_bytes(_lib.RDB_OP_LINEAR_BWD_PROJECTED_TO, ref)
+    ws = torch.randint(0, 256, (need + 64,), dtype=torch.uint8, device="cuda")
+    tail = ws[need:].clone()
+    dx, got = (torch.full((T, in_f), 7.0, dtype=bf, device="cuda") for _ in range(2))
+    dc, dc2 = torch.empty_like(c), torch.empty_like(c)
+    assert lib.rdb_linear_bwd_projected_to(dx.data_ptr(), in_f, dc.data_ptr(), 1, dy.data_ptr(), out_f, state.data_ptr(), c.data_ptr(), ref, ws.data_ptr(), need, stream) == 0
+    leaf = h.clone().requires_grad_()
+    want, = torch.autograd.grad(_lib.extension().relu_square(leaf), leaf, dx)
+    assert lib.rdb_linear_bwd_projected_relu_square(got.data_ptr(), dc2.data_ptr(), dy.data_ptr(), out_f, state.data_ptr(), c.data_ptr(), h.data_ptr(), ref, ws.data_ptr(),
+                                                    need, stream) == 0
+    same = lambda a, b: torch.equal(torch.nan_to_num(a, nan=1234.0), torch.nan_to_num(b, nan=1234.0))
+    assert same(got, want) and same(dc2, dc) and torch.equal(ws[need:], tail)
+    assert lib.rdb_linear_bwd_projected_relu_square(got.data_ptr() + 16, dc2.data_ptr(), dy.data_ptr(), out_f, state.data_ptr(), c.data_ptr(), h.data_ptr(), ref, ws.data_ptr(),
+                                                    need, stream) != 0
+
+
+@pytest.mark.parametrize("T,in_f,out_f,k", [(64, 72, 64, 64), (512, 128, 64, 264)])
+def test_layers_whose_dx_has_no_such_store(T, in_f, out_f, k):
+    import ctypes
+
+    from randumb_amd import _lib, hip
+
+    c = torch.zeros(out_f, k, dtype=torch.bfloat16, device="cuda")
+    d = hip._desc(T, in_f, out_f, c, in_f, 1, 5, torch.bfloat16, 0)
+    assert _lib.load().rdb_linear_bwd_projected_takes_relu_square(ctypes.byref(d)) == 0

@@ -90,6 +90,8 @@ EXPORTS = [
     "rdb_rms_norm_fwd",
     "rdb_rms_norm_bwd",
     "rdb_relu_square",
+    "rdb_embedding_bwd_takes",
+    "rdb_embedding_bwd",
     "rdb_cross_entropy_fwd",
     "rdb_cross_entropy_bwd",
     "rdb_causal_attention_scratch_floats",
@@ -242,6 +244,10 @@ def load() -> ctypes.CDLL:
     L.rdb_linear_fwd_kept_pseudo_bias.restype = ci
     L.rdb_linear_fwd_kept_ws.argtypes = [vp, i64, vp, vp, i64, vp, vp, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_fwd_kept_ws.restype = ci
+    L.rdb_embedding_bwd_takes.argtypes = [i64, i64, i64]
+    L.rdb_embedding_bwd_takes.restype = ci
+    L.rdb_embedding_bwd.argtypes = [vp, vp, ci, vp, i64, i64, i64, vp]
+    L.rdb_embedding_bwd.restype = ci
     L.rdb_linear_bwd_projected_takes_relu_square.argtypes = [dp]
     L.rdb_linear_bwd_projected_takes_relu_square.restype = ci
     L.rdb_linear_bwd_projected_relu_square.argtypes = [vp, vp, vp, i64, vp, vp, vp, dp, vp, i64, vp]

@@ -1005,6 +1005,32 @@ class ReluSquare : public Function<ReluSquare> {
     }
 };
 
+// rows idx of a dense bf16 table; the gradient is the table's, in one launch
+class EmbedDense : public Function<EmbedDense> {
+  public:
+    static Tensor forward(AutogradContext *ctx, const Tensor &weight, const Tensor &idx)
+    {
+        ctx->save_for_backward({idx});
+        ctx->saved_data["m"] = std::vector<int64_t>{weight.size(0), weight.size(1), idx.numel()};
+        return at::embedding(weight, idx);
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const Tensor idx0 = ctx->get_saved_variables()[0];
+        const auto m = ctx->saved_data["m"].toIntVector();
+        constexpr const char *who = "embedding (backward)";
+        restored(who, idx0, grads[0], grads[0].sizes().slice(0, grads[0].dim() - 1));
+        if (at::GradMode::is_enabled() || grads[0].scalar_type() != at::kBFloat16 || (idx0.scalar_type() != at::kLong && idx0.scalar_type() != at::kInt))
+            return {at::embedding_dense_backward(grads[0], idx0, m[0], -1, false), Tensor()};
+        const Tensor idx = idx0.contiguous(), dy = dense(grads[0]);
+        restored_values(who, idx, dy, idx.scalar_type(), m[2]);
+        const c10::OptionalDeviceGuard guard(dy.device());
+        Tensor dw = at::empty({m[0], m[1]}, dy.options());
+        check(rdb_embedding_bwd(dw.data_ptr(), idx.data_ptr(), (int)idx.element_size(), dy.data_ptr(), m[2], m[0], m[1], stream_of(dy)), "rdb_embedding_bwd");
+        return {dw, Tensor()};
+    }
+};
+
 // mean cross entropy of bf16 logits (rows, classes), computed in fp32
 class CrossEntropy : public Function<CrossEntropy> {
   public:
@@ -1319,6 +1345,21 @@ PyObject *py_relu_square(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
 }
 
+// embedding(weight, idx): rows of a dense bf16 table; None without a backward pass to come, or for sizes that its kernel does not take
+PyObject *py_embedding(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 2);
+        const Tensor &w = tensor_arg(a[0]), &idx = tensor_arg(a[1]);
+        if (!past_dispatcher({&w, &idx}) || !at::GradMode::is_enabled() || !w.requires_grad()) Py_RETURN_NONE;
+        need_bf16("embedding", w);
+        same_device("embedding", w, {&idx});
+        if (w.dim() != 2 || !idx.dim() || (idx.scalar_type() != at::kLong && idx.scalar_type() != at::kInt) || !rdb_embedding_bwd_takes(idx.numel(), w.size(0), w.size(1)))
+            Py_RETURN_NONE;
+        return THPVariable_Wrap(EmbedDense::apply(w, idx));
+    });
+}
+
 // cross_entropy(logits, target, ignore_index): mean over the rows that count
 PyObject *py_cross_entropy(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
@@ -1374,6 +1415,7 @@ PyObject *py_set_hooks(PyObject *, PyObject *const *a, Py_ssize_t n)
 PyMethodDef methods[] = {RDB_METHOD(takes_projected),   RDB_METHOD(linear_projected), RDB_METHOD(linear_one_call), RDB_METHOD(relu_square_linear),
                          RDB_METHOD(linear_vector),     RDB_METHOD(embed_rows),       RDB_METHOD(set_hooks),
                          RDB_METHOD(rms_norm),          RDB_METHOD(add_rms_norm),     RDB_METHOD(relu_square),
+                         RDB_METHOD(embedding),
                          RDB_METHOD(cross_entropy),     RDB_METHOD(causal_attention), RDB_METHOD(once_differentiable),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_rdb_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -180,7 +180,19 @@ class RT_Block(nn.Module):
 
 
 # as they stand here: replaced ones are called
-_BLOCK_FORWARD, _LINEAR_FORWARD, _MODULE_CALL = RT_Block.forward, RT_CastedLinear.forward, nn.Module.__call__
+_BLOCK_FORWARD, _LINEAR_FORWARD, _EMBEDDING_FORWARD, _MODULE_CALL = RT_Block.forward, RT_CastedLinear.forward, nn.Embedding.forward, nn.Module.__call__
+
+
+def _embed(wte: nn.Module, idx: torch.Tensor) -> torch.Tensor:
+    """``wte(idx)``; of a plain table with a gradient of one launch (stock, a sort of the indices and a dozen small ones)."""
+    if type(wte) is nn.Embedding and nn.Embedding.forward is _EMBEDDING_FORWARD and _unhooked(wte) and torch.is_grad_enabled() and type(idx) in _PLAIN:
+        w = wte._parameters.get("weight")
+        if w is not None and wte.padding_idx is None and wte.max_norm is None and not (wte.scale_grad_by_freq or wte.sparse) and idx.is_cuda and not ops._tracing():
+            ext = _fused(w)
+            y = None if ext is None else ext.embedding(w, idx)
+            if y is not None:
+                return y
+    return wte(idx)
 
 
 class RT_GPT(nn.Module):
@@ -199,7 +211,7 @@ class RT_GPT(nn.Module):
             self.lm_head = nn.Linear(config.n_embd, config.vocab_size, bias=False)
 
     def forward(self, idx: torch.Tensor, target: torch.Tensor) -> torch.Tensor:
-        x = self.wte(idx)
+        x = _embed(self.wte, idx)
         x = RT_norm(x.to(self.h[0].mlp.c_fc.weight_coef.dtype))
         normed = None   # RT_norm(x) where it is at hand
         for block in self.h:

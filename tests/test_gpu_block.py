@@ -349,3 +349,33 @@ def test_squared_relu_in_the_projections_node(dim, k, tokens, kind):
     assert len(seen) == 1 and torch.equal(y, y2) and all(torch.equal(a, b) for a, b in zip(grads, grads2))
     node = lambda t: t.grad_fn.next_functions[0][0].next_functions[0][0]
     assert not torch.is_grad_enabled() or kind == "frozen input" or "ReluSquare" not in str(node(y)) and "ReluSquare" in str([node(y2)] + [f[0] for f in node(y2).next_functions])
+
+
+# one position, one row; fewer positions than waves; a last block of one row; rows of more than a wave's share (65, all, and half of the positions); columns of one
+# piece, of a part of one and of several
+@pytest.mark.parametrize("positions,vocab,dim,hot", [(1, 1, 8, 0), (7, 129, 64, 0), (600, 65, 520, 0), (1000, 64, 768, 65), (8192, 5030, 768, 4096), (3000, 40, 1032, 3000),
+                                                     (16384, 50304, 256, 64)])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_gradient_of_a_dense_table(ext, positions, vocab, dim, hot, dtype):
+    print(f"case dense table {positions} of {vocab} x {dim}, {hot} of them one row, {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(positions)
+    idx = torch.randint(0, vocab, (positions,), generator=g, device="cuda")
+    idx[torch.randperm(positions, generator=g, device="cuda")[:hot]] = vocab // 2
+    idx, w, dy = idx.to(dtype), bf16(g, vocab, dim).requires_grad_(), bf16(g, positions, dim)
+    y = ext.embedding(w, idx)
+    assert torch.equal(y, F.embedding(idx, w))
+    got, = torch.autograd.grad(y, w, dy)
+    want = torch.zeros(vocab, dim, dtype=torch.float64, device="cuda").index_add_(0, idx.long(), dy.double())
+    size = torch.zeros(vocab, dim, dtype=torch.float64, device="cuda").index_add_(0, idx.long(), dy.double().abs())
+    # bf16's rounding of the result, and at most `positions` roundings to 24 bits of sums no larger than `size`
+    assert bool(((got.double() - want).abs() <= 2.0**-8 * want.abs() + min(positions, 64 + positions / 8) * 2.0**-24 * size).all())
+    assert torch.equal(torch.autograd.grad(ext.embedding(w, idx), w, dy)[0], got)
+
+
+def test_dense_tables_that_the_kernel_leaves(ext):
+    w, many = torch.zeros(10, 64, device="cuda", dtype=torch.bfloat16, requires_grad=True), torch.zeros(16385, dtype=torch.int64, device="cuda")
+    assert ext.embedding(w, many) is None and ext.embedding(w, many[:0]) is None and ext.embedding(w.detach(), many[:5]) is None
+    assert ext.embedding(torch.zeros(10, 60, device="cuda", dtype=torch.bfloat16, requires_grad=True), many[:5]) is None
+    y = ext.embedding(w, many[:6].view(2, 3))
+    g, = torch.autograd.grad(y, w, torch.ones_like(y).requires_grad_(), create_graph=True)
+    assert g.requires_grad and float(g[0, 0]) == 6.0 and float(g[1:].abs().sum()) == 0.0

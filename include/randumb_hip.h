@@ -408,6 +408,10 @@ int rdb_linear_bwd_projected_rbias(void *dx, int64_t lddx, void *dcoef, int dcoe
                                    const void *scale_bias, const rdb_linear_desc *desc, void *workspace, int64_t workspace_bytes,
                                    void *stream);
 
+/* rdb_linear_project_fwd_ws of a bf16 layer without a bias, and square = relu(y)^2; both [tokens x out_f], contiguous, square 16-byte aligned. */
+int rdb_linear_project_fwd_relu_square(void *y, void *square, void *state, const void *x, int64_t ldx, const void *coef,
+                                       const rdb_linear_desc *desc, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* rdb_linear_bwd_projected_to (dcoef in bf16) of a layer whose input was the squared ReLU of `gate` ([tokens x in_f] bf16, contiguous, as dx is): dx is the
  * gradient of `gate`, that of the layer's input, in bf16, times 2 relu(gate), in the pass that stores it.  For the layers of which the first call says 1 (bf16, one
  * chunk of tokens, k <= 256, in_f a multiple of 64); dx 128-byte aligned, gate 16-byte aligned; workspace as rdb_linear_bwd_projected_to. */

@@ -76,6 +76,7 @@ EXPORTS = [
     "rdb_linear_fwd_kept",
     "rdb_linear_fwd_kept_pseudo_bias",
     "rdb_linear_fwd_kept_ws",
+    "rdb_linear_project_fwd_relu_square",
     "rdb_linear_bwd_projected_takes_relu_square",
     "rdb_linear_bwd_projected_relu_square",
     "rdb_linear_bwd_kept",
@@ -244,6 +245,8 @@ def load() -> ctypes.CDLL:
     L.rdb_linear_fwd_kept_pseudo_bias.restype = ci
     L.rdb_linear_fwd_kept_ws.argtypes = [vp, i64, vp, vp, i64, vp, vp, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_fwd_kept_ws.restype = ci
+    L.rdb_linear_project_fwd_relu_square.argtypes = [vp, vp, vp, vp, i64, vp, dp, vp, i64, vp]
+    L.rdb_linear_project_fwd_relu_square.restype = ci
     L.rdb_embedding_bwd_takes.argtypes = [i64, i64, i64]
     L.rdb_embedding_bwd_takes.restype = ci
     L.rdb_embedding_bwd.argtypes = [vp, vp, ci, vp, i64, i64, i64, vp]

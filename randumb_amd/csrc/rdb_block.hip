@@ -126,13 +126,6 @@ template <int NV, bool ADD> __global__ __launch_bounds__(256) void rms_norm_bwd_
 
 // ----------------------------------------------------------------------------------------------- squared ReLU
 // y = relu(x)^2;  dx = dy * 2 relu(x).  Memory bound: 16 bytes a lane and step, two steps in flight.
-__device__ __forceinline__ float relu(float v) { return v <= 0.0f ? 0.0f : v; }   // NaN stays NaN
-__device__ __forceinline__ uint32_t relu2_pair(uint32_t w)
-{
-    const float a = relu(lo_f32(w)), b = relu(hi_f32(w));
-    return f32x2_to_bf16x2(a * a, b * b);
-}
-
 template <bool GRAD> __global__ __launch_bounds__(256) void relu_square_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ x,
                                                                                const bf16_t *__restrict__ dy, int64_t n)
 {

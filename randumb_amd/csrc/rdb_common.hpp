@@ -135,6 +135,12 @@ __device__ __forceinline__ bf16_t f32_to_bf16(float f) { return (bf16_t)(f32x2_t
 // two bf16 values in a word
 __device__ __forceinline__ float lo_f32(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float hi_f32(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
+__device__ __forceinline__ float relu(float v) { return v <= 0.0f ? 0.0f : v; }   // NaN stays NaN
+__device__ __forceinline__ uint32_t relu2_pair(uint32_t w)
+{
+    const float a = relu(lo_f32(w)), b = relu(hi_f32(w));
+    return f32x2_to_bf16x2(a * a, b * b);
+}
 // the gradient of relu(x)^2, d * 2 relu(x), of two values: 0 where x <= 0 whatever d is, an infinite or undefined one included
 __device__ __forceinline__ uint32_t relu2_grad_pair(uint32_t x, uint32_t d)
 {

@@ -312,11 +312,11 @@ struct BwdBsParams {
     int tn_blocks;
 };
 
-template <int KG, int AUX, bool TABLE, bool GATE = false> __global__ __launch_bounds__(ST_THREADS, 1) void bwd_tns_red_kernel(BwdBsParams p)
+template <int KG, int AUX, bool TABLE, int SIDE = ST_ALONE> __global__ __launch_bounds__(ST_THREADS, 1) void bwd_tns_red_kernel(BwdBsParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     if ((int)blockIdx.x < p.tn_blocks)
-        stationary_block<KG, false, !TABLE, AUX, true, TABLE, GATE>(p.tn, smem_raw, blockIdx.x);
+        stationary_block<KG, false, !TABLE, AUX, true, TABLE, SIDE>(p.tn, smem_raw, blockIdx.x);
     else
         red_block(p.red, blockIdx.x - p.tn_blocks, gridDim.x - p.tn_blocks);
 }
@@ -593,12 +593,12 @@ int linear_bwd_projected(void *dx, int64_t lddx, float *dcoef, const void *dy, i
             if (rblocks < 1) rblocks = 1;
             if (direct) rblocks = 0;
             bs.tn.coef = n;
-            bs.tn.gate = static_cast<const bf16_t *>(gate);
+            bs.tn.side = static_cast<bf16_t *>(const_cast<void *>(gate));   // read
             return with_stationary_variant(bs.tn, [&](auto kg, auto aux) {
                 constexpr int KG = decltype(kg)::value, AUX = decltype(aux)::value;
                 auto kernel = n ? bwd_tns_red_kernel<KG, AUX, (KG > 2)> : bwd_tns_red_kernel<KG, AUX, false>;   // no table up to k = 128
                 if constexpr (AUX == Y_STREAM)
-                    if (gate) kernel = n ? bwd_tns_red_kernel<KG, AUX, (KG > 2), true> : bwd_tns_red_kernel<KG, AUX, false, true>;
+                    if (gate) kernel = n ? bwd_tns_red_kernel<KG, AUX, (KG > 2), ST_GATE> : bwd_tns_red_kernel<KG, AUX, false, ST_GATE>;
                 const size_t smem_s = stationary_smem(kg);
                 if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem_s, "bwd_tns_red_kernel")) return rl;
                 kernel<<<bs.tn_blocks + rblocks, ST_THREADS, smem_s, s>>>(bs);

@@ -432,7 +432,7 @@ struct ZYParams {
     StParams y;
 };
 
-template <int KG, bool BIAS, int AUX> __global__ __launch_bounds__(ST_THREADS, 1) void factored_zy_kernel(ZYParams p)
+template <int KG, bool BIAS, int AUX, int SIDE = ST_ALONE> __global__ __launch_bounds__(ST_THREADS, 1) void factored_zy_kernel(ZYParams p)
 {
     static_assert(KZ_THREADS == ST_THREADS && KZ_BT == ST_BT, "one block size and one token tile for both kinds of block");
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -442,7 +442,7 @@ template <int KG, bool BIAS, int AUX> __global__ __launch_bounds__(ST_THREADS, 1
     else if (block < p.z.c_blocks)
         transpose_units(p.z, block * (KZ_THREADS / 64) + (int)(threadIdx.x >> 6), p.z.c_blocks * (KZ_THREADS / 64));
     else
-        stationary_block<KG, BIAS, false, AUX, true>(p.y, smem_raw, block - p.z.c_blocks);
+        stationary_block<KG, BIAS, false, AUX, true, false, SIDE>(p.y, smem_raw, block - p.z.c_blocks);
 }
 
 // ----------------------------------------------------------------------------------------------- dC = dy^T . z
@@ -656,6 +656,8 @@ template <bool BIAS> static int launch_zy(const ZYParams &p, int y_items, hipStr
 {
     return with_stationary_variant(p.y, [&](auto kg, auto aux) {
         auto kernel = factored_zy_kernel<decltype(kg)::value, BIAS, decltype(aux)::value>;
+        if constexpr (!BIAS && decltype(aux)::value == Y_STREAM)
+            if (p.y.side) kernel = factored_zy_kernel<decltype(kg)::value, BIAS, decltype(aux)::value, ST_SQUARE>;
         const size_t smem = std::max(z_smem(), stationary_smem(kg));
         if (int rl = reserve_lds(reinterpret_cast<const void *>(kernel), smem, "factored_zy_kernel")) return rl;
         kernel<<<p.z.z_grid + p.z.c_blocks + xcd_grid_size(y_items), ST_THREADS, smem, s>>>(p);
@@ -673,8 +675,9 @@ template <bool BIAS> static int launch_ys(const StParams &q, int items, hipStrea
 // state <- projection of x (with the transposed coefficients if with_ct), y <- forward product, in one launch when the
 // contraction of a token fits in registers (k <= 256), otherwise in two.
 // polls: how long its multiplying blocks wait; fewer than SYNC_SPIN_LIMIT in a self-test only.
+// square: NULL, or *square where relu(y)^2 goes, laid out as y is; *square becomes NULL where it is written (one launch, whole lines of y, no bias).
 int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, bool with_ct, const void *bias,
-                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls, void *scratch, int64_t scratch_bytes)
+                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls, void *scratch, int64_t scratch_bytes, void **square)
 {
     ZYParams p;
     if (!fill_z_params(p.z, state, x, ldx, with_ct ? coef : nullptr, d)) return RDB_E_UNSUPPORTED;
@@ -699,6 +702,10 @@ int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t
     const bool spread = spread_ranges(p.z, state, y, ldy, d, enough_scratch(scratch, scratch_bytes, d), &rc);
     if (rc) return rc;
     set_z_grid(p.z, xcd_grid_size(p.z.tiles_m * p.z.tiles_t) * (spread ? p.z.ranges : 1), num_cus);
+    if (square && !bias && ldy % 64 == 0 && ((uintptr_t)y & 127) == 0 && aligned16(*square)) {
+        p.y.side = static_cast<bf16_t *>(*square);
+        *square = nullptr;
+    }
     return bias ? launch_zy<true>(p, y_items, s) : launch_zy<false>(p, y_items, s);
 }
 
@@ -772,7 +779,7 @@ int linear_fwd_factored(void *y, int64_t ldy, const void *x, int64_t ldx, const 
     if (((uintptr_t)bias & 7) || d->tokens * ldy >= (1ll << 29)) return RDB_E_UNSUPPORTED;
     const int64_t state = linear_projection_bytes(d);   // a multiple of 256; the scratch lies behind it
     return linear_project_fwd(y, ldy, workspace, x, ldx, coef, false, bias, d, num_cus, s, SYNC_SPIN_LIMIT, static_cast<char *>(workspace) + state,
-                              workspace_bytes - state);
+                              workspace_bytes - state, nullptr);
 }
 
 // dC = dy^T . (x . N^T) with the projection state in the workspace; dcoef must have been zeroed on the same stream.

@@ -290,7 +290,7 @@ int64_t linear_projection_scratch(const rdb_linear_desc *d);
 int linear_project(void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d, hipStream_t s, void *scratch = nullptr,
                    int64_t scratch_bytes = 0);
 int linear_project_fwd(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, bool with_ct, const void *bias,
-                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls = SYNC_SPIN_LIMIT, void *scratch = nullptr, int64_t scratch_bytes = 0);
+                       const rdb_linear_desc *d, int num_cus, hipStream_t s, int polls = SYNC_SPIN_LIMIT, void *scratch = nullptr, int64_t scratch_bytes = 0, void **square = nullptr);
 int linear_fwd_projected(void *y, int64_t ldy, const void *z, const void *coef, const void *bias, const rdb_linear_desc *d, int num_cus,
                          hipStream_t s);
 int linear_dcoef_projected(float *dcoef, const void *dy, int64_t lddy, const void *z, const rdb_linear_desc *d, int num_cus, hipStream_t s);
@@ -1163,8 +1163,8 @@ extern "C" int rdb_linear_project_fwd(void *y, int64_t ldy, void *state, const v
     return rdb_linear_project_fwd_ws(y, ldy, state, x, ldx, coef, bias, d, nullptr, 0, stream);
 }
 
-extern "C" int rdb_linear_project_fwd_ws(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, const void *bias,
-                                         const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
+static int project_fwd_entry(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, const void *bias, const rdb_linear_desc *d, void *workspace,
+                             int64_t workspace_bytes, void *stream, void **square)
 {
     if (f32_projected(d)) {
         if (int rc = check_projected_f32("rdb_linear_project_fwd", d)) return rc;
@@ -1188,11 +1188,27 @@ extern "C" int rdb_linear_project_fwd_ws(void *y, int64_t ldy, void *state, cons
         const rdb_linear_desc dd = chunk_desc(d, pl, c);
         rc = linear_project_fwd(at_bytes(y, c * pl.chunk_tokens * ldy * 2), ldy, at_bytes(state, c * pl.state_stride),
                                 at_bytes(x, c * pl.chunk_tokens * ldx * 2), ldx, coef, true, bias, &dd, num_compute_units(), (hipStream_t)stream,
-                                SYNC_SPIN_LIMIT, workspace, workspace_bytes);
+                                SYNC_SPIN_LIMIT, workspace, workspace_bytes, pl.nchunks == 1 ? square : nullptr);
         if (rc == RDB_E_UNSUPPORTED) return set_error(RDB_E_UNSUPPORTED, "rdb_linear_project_fwd: internal: chunk %d of %d refused", c, pl.nchunks);
         if (rc) return rc;
     }
     return RDB_OK;
+}
+
+extern "C" int rdb_linear_project_fwd_ws(void *y, int64_t ldy, void *state, const void *x, int64_t ldx, const void *coef, const void *bias,
+                                         const rdb_linear_desc *d, void *workspace, int64_t workspace_bytes, void *stream)
+{
+    return project_fwd_entry(y, ldy, state, x, ldx, coef, bias, d, workspace, workspace_bytes, stream, nullptr);
+}
+
+extern "C" int rdb_linear_project_fwd_relu_square(void *y, void *square, void *state, const void *x, int64_t ldx, const void *coef, const rdb_linear_desc *d,
+                                                  void *workspace, int64_t workspace_bytes, void *stream)
+{
+    if (!d || !square) return set_error(RDB_E_NULL, "rdb_linear_project_fwd_relu_square: desc or square is NULL");
+    if (d->act_dtype != RDB_BF16 || !aligned16(square)) return set_error(RDB_E_UNSUPPORTED, "rdb_linear_project_fwd_relu_square: bf16 layers, square 16-byte aligned");
+    void *left = square;
+    if (int rc = project_fwd_entry(y, d->out_f, state, x, ldx, coef, nullptr, d, workspace, workspace_bytes, stream, &left)) return rc;
+    return left ? rdb_relu_square(square, y, nullptr, d->tokens * d->out_f, stream) : RDB_OK;
 }
 
 static int64_t project_fwd_rbias_table(const rdb_linear_desc *d)

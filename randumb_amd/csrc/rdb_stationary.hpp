@@ -25,6 +25,7 @@ constexpr int Y_STREAM = 2;
 
 constexpr int ST_BT = 256, ST_BO = 64, ST_STG_LD = ST_BO + 8, ST_WAVES = 8, ST_THREADS = ST_WAVES * 64, ST_TW = ST_BT / ST_WAVES;
 constexpr int ST_KMAX = 256;
+constexpr int ST_ALONE = 0, ST_GATE = 1, ST_SQUARE = 2;
 
 struct StParams {
     const bf16_t *z;     // left operand [tokens x k]: row-major, or (ZFRAG) in fragment order as store_tile_bf16_frag writes it,
@@ -32,7 +33,7 @@ struct StParams {
     const bf16_t *coef;  // right operand [out_f x k], or (TABLE) in fragment order; not used when the right operand is noise
     const bf16_t *bias;  // [out_f] or NULL
     bf16_t *y;           // [tokens x out_f], leading dimension ldy
-    const bf16_t *gate;  // GATE: as y is
+    bf16_t *side;        // ST_GATE, ST_SQUARE: as y is
     int64_t ldy;
     int tokens, out_f, k;
     int tiles_t, splits, units_per_split;
@@ -50,10 +51,11 @@ struct StParams {
 // (exact in bf16).  AUX: cache policy of the row stores (an immediate of the instruction: two copies of the steps in one kernel cost it 10 to 20
 // registers, and spills with k = 256 and a bias).
 // TABLE: `coef` is in fragment order (rows padded to 32, k to kpad, zeros there): a unit's tile is consecutive kilobytes.
-// GATE: the rows leave as y * 2 relu(gate) (relu2_grad_pair of their bf16 values), the input gradient of a layer behind a squared ReLU: the product's
-// rows are not written, read again and written.  A unit's pieces of gate are loaded in its own step and used a step later, behind a unit's matrix
+// SIDE, ST_GATE: the rows leave as y * 2 relu(side) (relu2_grad_pair of their bf16 values), the input gradient of a layer behind a squared ReLU: the product's
+// rows are not written, read again and written.  A unit's pieces of side are loaded in its own step and used a step later, behind a unit's matrix
 // instructions, which also cover the arithmetic (200 vector instructions a wave and unit beside 32 matrix instructions).
-template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE, bool GATE> struct StBlock {
+// ST_SQUARE: side = relu(y)^2 is written beside y, for the layer behind it, with plain stores: it is read next.
+template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE, int SIDE> struct StBlock {
     static constexpr int kpad = KG * 64, ldk = kpad + 8, cpr = kpad / 8, ncp = ST_BO * cpr, NQ = ncp / ST_THREADS;
     const StParams &p;
     bf16_t *Cs;   // [2][64 rows][ldk]
@@ -66,7 +68,7 @@ template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE, bool GATE> struct 
     uint2 braw[2][4];   // bias of the unit whose epilogue comes next: four output features per (mi, jq) of this lane
     int tok_y;          // token of the row piece this lane stores in step 0 of the epilogue; step q: 8 q further
     uint32_t off_y;     // its byte offset in y at output feature 0
-    u32x4 graw[GATE ? 4 : 1];   // gate of the unit whose epilogue comes next, as the row pieces of y
+    u32x4 graw[SIDE == ST_GATE ? 4 : 1];   // gate of the unit whose epilogue comes next, as the row pieces of y
 
     __device__ __forceinline__ void issue(int unit)
     {   // global -> registers for a C tile; rows past out_f read as zeros
@@ -146,7 +148,7 @@ template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE, bool GATE> struct 
             return at + (lane & 7) * 8 < p.out_f && tok_y + qq * 8 < p.tokens ? off_y + (uint32_t)(qq * 8 * (int)p.ldy * 2 + at * 2) : BUFFER_OOB;
         };
         u32x4 gnow[4];
-        if constexpr (GATE) {
+        if constexpr (SIDE == ST_GATE) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 gnow[q] = graw[q];
@@ -176,7 +178,7 @@ template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE, bool GATE> struct 
 #pragma unroll
                 for (int q = 0; q < 2; ++q) {
                     const int qq = h * 2 + q;
-                    if constexpr (GATE) {
+                    if constexpr (SIDE == ST_GATE) {
                         u32x4 d = __builtin_bit_cast(u32x4, v[q]);
 #pragma unroll
                         for (int i = 0; i < 4; ++i) d[i] = relu2_grad_pair(gnow[qq][i], d[i]);
@@ -184,6 +186,12 @@ template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE, bool GATE> struct 
                     }
                     const uint32_t a = piece(o0, qq);
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v[q]), rs_y, (int)a, 0, AUX);
+                    if constexpr (SIDE == ST_SQUARE) {
+                        u32x4 d = __builtin_bit_cast(u32x4, v[q]);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) d[i] = relu2_pair(d[i]);
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, d), rs_g, (int)a, 0, 0);
+                    }
                 }
                 if (op == 9) __builtin_amdgcn_wave_barrier();
             }
@@ -234,10 +242,10 @@ template <int KG, bool BIAS, bool NOISE, int AUX, bool TABLE, bool GATE> struct 
 };
 
 // `block`: index of this block among the blocks that run this body; all ST_THREADS threads of the block must call.
-template <int KG, bool BIAS, bool NOISE, int AUX, bool ZFRAG = false, bool TABLE = false, bool GATE = false>
+template <int KG, bool BIAS, bool NOISE, int AUX, bool ZFRAG = false, bool TABLE = false, int SIDE = ST_ALONE>
 __device__ __forceinline__ void stationary_block(const StParams &p, unsigned char *smem_raw, int block)
 {
-    typedef StBlock<KG, BIAS, NOISE, AUX, TABLE, GATE> B;
+    typedef StBlock<KG, BIAS, NOISE, AUX, TABLE, SIDE> B;
     const int t = threadIdx.x, wave = t >> 6;
     // work item = (token tile, split), split fastest: neighbours share the left operand's tile, everyone shares the right operand
     const int w = xcd_work_item(block, p.tiles_t * p.splits);
@@ -257,7 +265,7 @@ __device__ __forceinline__ void stationary_block(const StParams &p, unsigned cha
                                                NOISE ? 0 : TABLE ? (p.out_f + 31) / 32 * 32 * B::kpad * 2 : (int)((int64_t)p.out_f * p.k * 2), 0x00020000);
     b.rs_y = __builtin_amdgcn_make_buffer_rsrc(p.y, 0, (int)(((int64_t)(p.tokens - 1) * p.ldy + p.out_f) * 2), 0x00020000);
     b.rs_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(p.bias), 0, p.bias ? p.out_f * 2 : 0, 0x00020000);  // no bias: zeros
-    if constexpr (GATE) b.rs_g = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(p.gate), 0, (int)(((int64_t)(p.tokens - 1) * p.ldy + p.out_f) * 2), 0x00020000);
+    if constexpr (SIDE != ST_ALONE) b.rs_g = __builtin_amdgcn_make_buffer_rsrc(p.side, 0, (int)(((int64_t)(p.tokens - 1) * p.ldy + p.out_f) * 2), 0x00020000);
     b.t = t;
     if constexpr (ZFRAG) {
         // the fragments lie ready in memory, a k-step of a wave's 32 tokens in 1024 consecutive bytes: no staging, no barrier
@@ -285,6 +293,7 @@ __device__ __forceinline__ void stationary_block(const StParams &p, unsigned cha
                 for (int e = t; e < ST_BT * pieces; e += ST_THREADS) {
                     const int tok = (w / p.splits) * ST_BT + e / pieces, o = o_begin + (e % pieces) * 8;
                     if (tok < p.tokens) __builtin_amdgcn_raw_buffer_store_b128(nan8, b.rs_y, (int)(((int64_t)tok * p.ldy + o) * 2), 0, 0);
+                    if (SIDE == ST_SQUARE && tok < p.tokens) __builtin_amdgcn_raw_buffer_store_b128(nan8, b.rs_g, (int)(((int64_t)tok * p.ldy + o) * 2), 0, 0);
                 }
                 return;
             }
@@ -379,7 +388,7 @@ inline int make_stationary_grid(StParams &q, int64_t tokens, int64_t out_f, int 
 {
     q.tokens = (int)tokens;
     q.out_f = (int)out_f;
-    q.gate = nullptr;
+    q.side = nullptr;
     q.sync = nullptr;   // the left operand comes from an earlier launch unless the caller says otherwise afterwards
     q.sync_tag = 0;
     q.sync_n = 0;

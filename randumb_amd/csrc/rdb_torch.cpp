@@ -502,16 +502,17 @@ Tensor relu_squared(const Tensor &x, const Tensor &dy = Tensor());   // relu(x)^
 Tensor relu_squared_with_graph(const Tensor &x, const Tensor &dy);
 // The forward pass keeps z = x.N^T (and, in bf16, the transposed coefficients) for the backward pass, which needs nothing else
 // of x; with the fused random bias its full-rank share is added on top in both directions and x is saved as well.
-// squared: the layer's input is relu(x)^2, which nothing keeps, and its gradient goes through that on its way to memory (8192 tokens x 3072 -> 768, k = 256:
+// square: where relu(y)^2 is left beside y, for a layer of that input (or NULL).
+// squared: the layer's input is relu(x)^2, formed here unless `formed` is that, which nothing keeps, and its gradient goes through that on its way to memory (8192 tokens x 3072 -> 768, k = 256:
 // backward and a pass over its dx 62.8 us, 47.7 so).
 class ProjectedLinear : public Function<ProjectedLinear> {
   public:
     static Tensor forward(AutogradContext *ctx, const Tensor &x0, const Tensor &coefs, const OptTensor &bias, const OptTensor &bias_scale, int64_t bias_seed,
-                          const OptTensor &scale_bias, const Layer &l, bool squared)
+                          const OptTensor &scale_bias, const Layer &l, bool squared, const Tensor *formed = nullptr, Tensor *square = nullptr)
     {
         const Bias pb{bias, bias_scale, bias_seed};
         const c10::OptionalDeviceGuard guard(x0.device());
-        const Tensor x = squared ? relu_squared(x0) : near_act(x0), c = coefs.contiguous();
+        const Tensor x = !squared ? near_act(x0) : formed ? *formed : relu_squared(x0), c = coefs.contiguous();
         const rdb_linear_desc d = desc(x, l, c);
         const int64_t need = rdb_linear_projection_bytes(&d);
         Tensor state = bytes(need, x), y = at::empty({x.size(0), l.out_f}, x.options());
@@ -526,7 +527,9 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         } else {
             const int64_t room = rdb_linear_workspace_bytes(RDB_OP_LINEAR_PROJECT, &d);
             const Tensor ws = bytes(room, x);
-            check(rdb_linear_project_fwd_ws(y.data_ptr(), l.out_f, ptr(state), x.data_ptr(), x.stride(0), c.data_ptr(), ptr(b), &d, ptr(ws), room, s),
+            if (square) *square = at::empty_like(y);
+            check(square ? rdb_linear_project_fwd_relu_square(y.data_ptr(), square->data_ptr(), ptr(state), x.data_ptr(), x.stride(0), c.data_ptr(), &d, ptr(ws), room, s)
+                         : rdb_linear_project_fwd_ws(y.data_ptr(), l.out_f, ptr(state), x.data_ptr(), x.stride(0), c.data_ptr(), ptr(b), &d, ptr(ws), room, s),
                   "rdb_linear_project_fwd");
         }
         if (scale_bias && !one_product) {
@@ -551,7 +554,7 @@ class ProjectedLinear : public Function<ProjectedLinear> {
         gradients(ctx, grads, dx, dc, ds, db, m[6] && !graph);
         layer_gradients(grads[0], m[3] ? (int)(2 + m[4]) : -1, dx, dc, ds, db, ctx->saved_data["bias"].toIntVector());
         if (m[6] && graph && dx.defined()) dx = relu_squared_with_graph(ctx->get_saved_variables()[3], dx);
-        return {dx, dc, db.first, db.second, Tensor(), ds, Tensor(), Tensor()};
+        return {dx, dc, db.first, db.second, Tensor(), ds, Tensor(), Tensor(), Tensor(), Tensor()};
     }
     // through: dx is to be the gradient behind relu(x)^2
     static void gradients(AutogradContext *ctx, const variable_list &grads, Tensor &dx, Tensor &dc, Tensor &dsb, std::pair<Tensor, Tensor> &db, bool through)
@@ -1227,7 +1230,7 @@ PyObject *py_linear_projected(PyObject *, PyObject *const *a, Py_ssize_t n)
         // without a backward pass to come there is no state to keep: the one-call forward
         if (!at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad() || wants_grad(b) || wants_grad(sb)))
             return THPVariable_Wrap(linear_fwd(x, c, l, sb, b));
-        return THPVariable_Wrap(ProjectedLinear::apply(x, c, b.coef, b.scale, b.seed, sb, l, false));
+        return THPVariable_Wrap(ProjectedLinear::apply(x, c, b.coef, b.scale, b.seed, sb, l, false, (const Tensor *)nullptr, (Tensor *)nullptr));
     });
 }
 
@@ -1243,7 +1246,27 @@ PyObject *py_relu_square_linear(PyObject *, PyObject *const *a, Py_ssize_t n)
         check_sizes("linear_fwd", x, c, l, OptTensor(), Bias{});
         if (!past_dispatcher({&x, &c}) || !at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad())) Py_RETURN_NONE;
         need_bf16("relu_square_linear", x);
-        return THPVariable_Wrap(ProjectedLinear::apply(x, c, OptTensor(), OptTensor(), -1, OptTensor(), l, true));
+        return THPVariable_Wrap(ProjectedLinear::apply(x, c, OptTensor(), OptTensor(), -1, OptTensor(), l, true, (const Tensor *)nullptr, (Tensor *)nullptr));
+    });
+}
+
+// squared_relu_mlp(x, coefs 1, coefs 2, in_f, hidden, out_f, seed 1, seed 2): linear_projected, relu(.)^2 and linear_projected, each a node of its own but for the
+// activation, which is the second one's and leaves the first one's kernel beside its input; None as relu_square_linear
+PyObject *py_squared_relu_mlp(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        count_args(n, 8);
+        const Tensor &x = tensor_arg(a[0]), &c1 = tensor_arg(a[1]), &c2 = tensor_arg(a[2]);
+        const int64_t in_f = int_arg(a[3]), hidden = int_arg(a[4]), out_f = int_arg(a[5]);
+        const Layer l1{in_f, hidden, in_f, 1, seed_arg(a[6])}, l2{hidden, out_f, hidden, 1, seed_arg(a[7])};
+        same_device("linear_fwd", x, {&c1, &c2});
+        check_sizes("linear_fwd", x, c1, l1, OptTensor(), Bias{});
+        if (!past_dispatcher({&x, &c1, &c2}) || !at::GradMode::is_enabled() || !(x.requires_grad() || c1.requires_grad())) Py_RETURN_NONE;
+        need_bf16("squared_relu_mlp", x);
+        Tensor square;
+        const Tensor h = ProjectedLinear::apply(x, c1, OptTensor(), OptTensor(), -1, OptTensor(), l1, false, (const Tensor *)nullptr, &square);
+        check_sizes("linear_fwd", h, c2, l2, OptTensor(), Bias{});
+        return THPVariable_Wrap(ProjectedLinear::apply(h, c2, OptTensor(), OptTensor(), -1, OptTensor(), l2, true, (const Tensor *)&square, (Tensor *)nullptr));
     });
 }
 
@@ -1412,7 +1435,7 @@ PyObject *py_set_hooks(PyObject *, PyObject *const *a, Py_ssize_t n)
 }
 
 #define RDB_METHOD(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {RDB_METHOD(takes_projected),   RDB_METHOD(linear_projected), RDB_METHOD(linear_one_call), RDB_METHOD(relu_square_linear),
+PyMethodDef methods[] = {RDB_METHOD(takes_projected),   RDB_METHOD(linear_projected), RDB_METHOD(linear_one_call), RDB_METHOD(relu_square_linear), RDB_METHOD(squared_relu_mlp),
                          RDB_METHOD(linear_vector),     RDB_METHOD(embed_rows),       RDB_METHOD(set_hooks),
                          RDB_METHOD(rms_norm),          RDB_METHOD(add_rms_norm),     RDB_METHOD(relu_square),
                          RDB_METHOD(embedding),

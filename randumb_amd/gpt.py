@@ -125,6 +125,16 @@ def _unhooked(m: nn.Module) -> bool:
             and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks))
 
 
+def _plain_layer(m: nn.Module, x: torch.Tensor):
+    """(coefficients, seed) of a layer that is its forward's product in x's dtype and nothing else, or None."""
+    if not (type(m) is RT_CastedLinear and RT_CastedLinear.forward is _LINEAR_FORWARD and _unhooked(m)):
+        return None
+    w, coef = m._buffers.get("weight"), m._parameters.get("weight_coef")
+    if w is None or coef is None or w.fused_bias or m.bias is not None or not m.fused or x.dtype != w.dtype or ops._tracing():
+        return None
+    return coef, w.seed
+
+
 class RT_MLP(nn.Module):
     def __init__(self, dim: int, config: RT_GPTConfig):
         super().__init__()
@@ -132,6 +142,9 @@ class RT_MLP(nn.Module):
         self.c_proj = RT_CastedLinear(4 * dim, dim, config)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        y = self._in_two_nodes(x)
+        if y is not None:
+            return y
         h = self.c_fc(x)
         ext = _fused(h)
         if ext is None:
@@ -142,19 +155,37 @@ class RT_MLP(nn.Module):
         a = ext.relu_square(h)
         return self.c_proj(F.relu(h).square() if a is None else a)
 
+    def _in_two_nodes(self, x: torch.Tensor):
+        """With the activation's value from c_fc's kernel and its gradient from c_proj's; None where a layer is more than its forward."""
+        ext = _fused(x) if torch.is_grad_enabled() else None
+        f, p = None if ext is None else _plain_layer(self.c_fc, x), self.c_proj
+        if f is None:
+            return None
+        q = _plain_layer(p, x)
+        if q is None or p.in_features != self.c_fc.out_features:
+            return None
+        in_f, hidden, out_f = self.c_fc.in_features, p.in_features, p.out_features
+        if x.shape[-1] != in_f:
+            return None
+        x2 = x.reshape(-1, in_f)
+        # c_proj's is the same question of as many rows
+        if not (ext.takes_projected(x2, f[0], in_f, hidden, in_f, 1, None, None) and ext.takes_projected(x2, q[0], hidden, out_f, hidden, 1, None, None)):
+            return None
+        y = ext.squared_relu_mlp(x2, f[0], q[0], in_f, hidden, out_f, f[1], q[1])
+        return None if y is None else y.reshape(*x.shape[:-1], out_f)
+
     def _proj_of_relu_square(self, h: torch.Tensor, ext):
         """Both in one autograd node, whose backward pass needs no pass over memory of its own for the activation; None where the layer is
         more than its forward, or no backward pass is to come."""
         p = self.c_proj
-        if not (torch.is_grad_enabled() and type(p) is RT_CastedLinear and RT_CastedLinear.forward is _LINEAR_FORWARD and _unhooked(p)):
-            return None
-        w, coef, in_f, out_f = p._buffers.get("weight"), p._parameters.get("weight_coef"), p.in_features, p.out_features
-        if w is None or coef is None or w.fused_bias or p.bias is not None or not p.fused or h.dtype != w.dtype or h.shape[-1] != in_f or ops._tracing():
+        q = _plain_layer(p, h) if torch.is_grad_enabled() else None
+        in_f, out_f = p.in_features, p.out_features
+        if q is None or h.shape[-1] != in_f:
             return None
         x = h.reshape(-1, in_f)
-        if not ext.takes_projected(x, coef, in_f, out_f, in_f, 1, None, None):
+        if not ext.takes_projected(x, q[0], in_f, out_f, in_f, 1, None, None):
             return None
-        y = ext.relu_square_linear(x, coef, in_f, out_f, w.seed)
+        y = ext.relu_square_linear(x, q[0], in_f, out_f, q[1])
         return None if y is None else y.reshape(*h.shape[:-1], out_f)
 
 

@@ -344,9 +344,13 @@ def test_squared_relu_in_the_projections_node(dim, k, tokens, kind):
     y, grads = run()
     assert "Projected" in y.grad_fn.name() or "Projected" in y.grad_fn.next_functions[0][0].name()
     seen = []
+    hook = mlp.c_fc.register_forward_hook(lambda m, args, out: seen.append(out))   # the activation from its own kernel
+    y1, grads1 = run()
+    assert len(seen) == 1 and torch.equal(y, y1) and all(torch.equal(a, b) for a, b in zip(grads, grads1))
+    hook.remove()
     mlp.c_proj.register_forward_hook(lambda m, args, out: seen.append(args[0]))
     y2, grads2 = run()
-    assert len(seen) == 1 and torch.equal(y, y2) and all(torch.equal(a, b) for a, b in zip(grads, grads2))
+    assert len(seen) == 2 and torch.equal(y, y2) and all(torch.equal(a, b) for a, b in zip(grads, grads2))
     node = lambda t: t.grad_fn.next_functions[0][0].next_functions[0][0]
     assert not torch.is_grad_enabled() or kind == "frozen input" or "ReluSquare" not in str(node(y)) and "ReluSquare" in str([node(y2)] + [f[0] for f in node(y2).next_functions])
 
@@ -379,3 +383,28 @@ def test_dense_tables_that_the_kernel_leaves(ext):
     y = ext.embedding(w, many[:6].view(2, 3))
     g, = torch.autograd.grad(y, w, torch.ones_like(y).requires_grad_(), create_graph=True)
     assert g.requires_grad and float(g[0, 0]) == 6.0 and float(g[1:].abs().sum()) == 0.0
+
+
+# one to four groups of 64 coefficients and more, rows that are no whole lines (72), one launch and two, a last tile of tokens that is not full
+@pytest.mark.parametrize("T,in_f,out_f,k", [(1, 64, 64, 8), (300, 96, 192, 72), (513, 128, 320, 128), (700, 256, 1024, 192), (1025, 768, 3072, 256), (300, 64, 72, 64), (513, 128, 256, 320)])
+@pytest.mark.parametrize("one_launch", [1, 0])
+def test_squared_relu_beside_a_forward_product(T, in_f, out_f, k, one_launch):
+    import ctypes
+
+    from randumb_amd import _lib, hip
+
+    print(f"case squared ReLU beside a forward product {T} x {in_f} -> {out_f} k={k}", flush=True)
+    lib, stream, g = _lib.load(), torch.cuda.current_stream().cuda_stream, torch.Generator(device="cuda").manual_seed(T)
+    x, c = bf16(g, T, in_f), bf16(g, out_f, k)
+    x[T // 2, 3] = float("inf")
+    before = hip.set_one_launch(one_launch)
+    try:
+        want, state = hip.linear_project_fwd(x, c, 5, None)
+        d = hip._desc(T, in_f, out_f, c, in_f, 1, 5, torch.bfloat16, 0)
+        y, a = (torch.full((T + 1, out_f), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        assert lib.rdb_linear_project_fwd_relu_square(y.data_ptr(), a.data_ptr(), state.data_ptr(), x.data_ptr(), in_f, c.data_ptr(), ctypes.byref(d), None, 0, stream) == 0
+        same = lambda u, v: torch.equal(torch.nan_to_num(u, nan=1234.0), torch.nan_to_num(v, nan=1234.0))
+        assert same(y[:T], want) and same(a[:T], F.relu(want).square())
+        assert bool((y[T] == 7.0).all()) and bool((a[T] == 7.0).all())
+    finally:
+        hip.set_one_launch(before)

@@ -159,11 +159,12 @@ static int fg_launch_ranges(FgProduct q, int room, float *part, int64_t stride, 
 
 // Two such products that do not need each other, in one launch, and their sums in one: t = dy . C and dC = dy^T . z.
 int fg_launch_pair(const FgProduct &t, const FgProduct &dc, hipStream_t s);   // rdb_f32_pair.hip
-// dc_sum: dC's sum where it is left to the launch that comes next, dx = t . N, whose blocks leave compute units free: where t's ranges are one, so that no launch of sums is left, or dC's
-// partial matrices are long enough, 8 MB, for a few of the product's blocks to lose less than that launch does.  2048 tokens x 768 -> 3072, k = 256, 16 MB: sums 7.6 -> 4.8 us,
-// dx 12.5 -> 13.2, step 98.3 -> 96.1; 4097 x 1001 -> 999, k = 100 in bf16, 6 MB: sums 4.5 -> 4.2, dx 15.6 -> 16.7 with dC's beside it.
+// dc_sum: dC's sum where it is left to the launch that comes next, dx = t . N: where t's ranges are one, so that no launch of sums is left, or that product's tiles leave compute
+// units free and dC's partial matrices are long, 8 MB.  2048 tokens x 768 -> 3072, k = 256, 192 tiles, 16 MB: sums 7.6 -> 4.8 us, dx 12.5 -> 13.2, step 98.3 -> 96.1; 512 tiles, 4096 x
+// 1024 -> 8192, k = 128: sums 8.1 -> 5.3, dx 17.4 -> 20.0, step 208.6 -> 210.7; 256 tiles, 1024 x 4096 -> 4096, k = 256: 106.6 -> 108.0; 6 MB, 4097 x 1001 -> 999, k = 100 in bf16: sums 4.5 ->
+// 4.2, dx 15.6 -> 16.7.
 static int fg_launch_pair_ranges(FgProduct t, int t_room, float *t_part, int64_t t_stride, FgProduct dc, int dc_room, float *dc_part, int64_t dc_stride,
-                                 int num_cus, hipStream_t s, FgSum &dc_sum)
+                                 int num_cus, hipStream_t s, const rdb_linear_desc *d, FgSum &dc_sum)
 {
     const FgPairPlan plan = fg_plan_pair({t.M, dc.M}, {t.N, dc.N}, {t.K, dc.K}, num_cus, {t_room, dc_room}, t.a_es == 2);
     FgProduct *const q[2] = {&t, &dc};
@@ -184,7 +185,11 @@ static int fg_launch_pair_ranges(FgProduct t, int t_room, float *t_part, int64_t
         }
     }
     if (int rc = fg_launch_pair(t, dc, s)) return rc;
-    const bool beside = !sum[0].blocks || sum[1].n * sum[1].splits * 4 >= (8 << 20);
+    bool beside = !sum[0].blocks;
+    if (!beside && sum[1].n * sum[1].splits * 4 >= (8 << 20)) {
+        const FgPlan dx = fg_plan(d->tokens, d->in_f, d->k, num_cus, 1, FgGroups<FG_KCONT, FG_NOISE_I>::four);
+        beside = cdiv(d->tokens, dx.bm) * cdiv(d->in_f, FG_BN) < num_cus;
+    }
     dc_sum = beside ? sum[1] : FgSum{};
     return fg_launch_sums(sum[0], beside ? FgSum{} : sum[1], s);
 }
@@ -281,6 +286,7 @@ static int fg_dx_from_t(void *dx, int64_t lddx, const float *t, const rdb_linear
     FgProduct q = {t, d->k, d->tokens * d->k, nullptr, 0, 0, (float *)dx, lddx, nullptr, d->tokens, d->in_f, d->k, 0, 0, 0, 0, d->seed};
     q.out_bf16 = d->act_dtype == RDB_BF16;
     q.sum = sum;
+    if (sum.blocks) q.split = true;   // as it was when the sum was left
     q.bias_grad = bias;
     return fg_launch<FG_KCONT, FG_NOISE_I>(q, num_cus, s, "f32_gemm_kernel (dx = t . N)");
 }
@@ -306,7 +312,7 @@ static int fg_backward(void *dx, int64_t lddx, void *dcoef, int dcoef_dtype, con
         const int64_t zt = up256(d->tokens * d->k * 4) / 4;
         FgSum dc_sum;
         if (int rc = fg_launch_pair_ranges(fg_t(t, dy, lddy, coef, d), t_room(d, num_cus), t + zt, zt, fg_dc(dcoef, dcoef_dtype, dy, lddy, z, d),
-                                           room, dc_part, dc_stride, num_cus, s, dc_sum))
+                                           room, dc_part, dc_stride, num_cus, s, d, dc_sum))
             return rc;
         return fg_dx_from_t(dx, lddx, t, d, num_cus, s, dc_sum, bias);
     }

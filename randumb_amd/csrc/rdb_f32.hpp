@@ -94,9 +94,12 @@ struct FgParams {
     int64_t lddot;
     float *dot_part;            // with dotm: one value per block, in block order (x fastest, then y)
     FgValues values;            // FG_NOISE_M on the B side: formed by the last blocks along z
+};
+// ... of a launch that carries more than its product: a type of its own, since every launch waits for what it is given (150 bytes more in each of the five of a step: +1 us)
+struct FgCarried : FgParams {
     FgSum sum;                  // FG_NOISE_I on the B side: a sum that an earlier launch left to do, by the last blocks along z
     int sum_slices;
-    BiasGrad bias_grad;         // FG_NOISE_I on the B side, or two FG_MCONT: by the blocks before those
+    BiasGrad bias_grad;         // by the blocks before those
     int bias_slices;
 };
 
@@ -739,8 +742,8 @@ template <int BM, int G, int BSRC> constexpr int fg_min_waves()
 // The last launch of a backward pass, dx = t . N or dC = dy^T . z alone, carries the gradient of a pseudorandom bias where dy is small: a launch of its own is 6 us
 // of kernel and as much on the host (128 images through 784 -> 256 -> 10, k = 64, fp32: 18 launches a step, 16 without).
 constexpr bool fg_carries_bias(int asrc, int bsrc) { return bsrc == FG_NOISE_I || (asrc == FG_MCONT && bsrc == FG_MCONT); }
-template <int BM, int G, int ASRC, int BSRC, int EPI, bool VEC, bool SPLIT, int AES, int BES>
-__global__ __launch_bounds__(FG_THREADS * G, (fg_min_waves<BM, G, BSRC>())) void f32_gemm_kernel(FgParams p)
+template <int BM, int G, int ASRC, int BSRC, int EPI, bool VEC, bool SPLIT, int AES, int BES, bool CARRY = false>
+__global__ __launch_bounds__(FG_THREADS * G, (fg_min_waves<BM, G, BSRC>())) void f32_gemm_kernel(std::conditional_t<CARRY, FgCarried, FgParams> p)
 {
     __shared__ __align__(16) float lds[FgBlock<BM, G, ASRC, BSRC, VEC, SPLIT, AES, BES>::LDS];
     __shared__ int not_finite;   // some thread's sum is an infinity or a NaN
@@ -753,7 +756,7 @@ __global__ __launch_bounds__(FG_THREADS * G, (fg_min_waves<BM, G, BSRC>())) void
             return;
         }
     }
-    if constexpr (fg_carries_bias(ASRC, BSRC)) {
+    if constexpr (CARRY) {
         const unsigned sums = gridDim.z - (unsigned)p.sum_slices, products = sums - (unsigned)p.bias_slices;
         if (blockIdx.z >= products) {
             const bool sum = BSRC == FG_NOISE_I && blockIdx.z >= sums;
@@ -954,6 +957,12 @@ struct FgProduct {
         const int nt = FG_THREADS * G_;                                                                             \
         auto of = [&](auto aes_, auto bes_) {                                                                       \
             constexpr int AES = decltype(aes_)::value, BES = decltype(bes_)::value;                                 \
+            if constexpr (fg_carries_bias(ASRC, BSRC) && EPI_ == FG_STORE)                                          \
+                if (more) {                                                                                         \
+                    if (vec) f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, true, true, AES, BES, true><<<grid, nt, 0, s>>>(carried); \
+                    else f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, false, true, AES, BES, true><<<grid, nt, 0, s>>>(carried);    \
+                    return;                                                                                         \
+                }                                                                                                   \
             if (vec) f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, true, true, AES, BES><<<grid, nt, 0, s>>>(p);       \
             else f32_gemm_kernel<BM_, G_, ASRC, BSRC, EPI_, false, true, AES, BES><<<grid, nt, 0, s>>>(p);          \
         };                                                                                                          \
@@ -1018,8 +1027,6 @@ inline FgParams fg_params(const FgProduct &q)
     p.lddot = q.lddot;
     p.dot_part = q.dot_part;
     p.values = q.values;
-    p.sum = q.sum;
-    p.bias_grad = q.bias_grad;
     return p;
 }
 // 16-byte pieces (8 of a bf16 matrix: four values) when both matrices allow them: aligned bases and leading dimensions, and the extent
@@ -1042,20 +1049,27 @@ template <int ASRC, int BSRC> int fg_launch(FgProduct q, int num_cus, hipStream_
     }
     if (!fg_fits(q)) return RDB_E_UNSUPPORTED;
     if constexpr (BSRC == FG_NOISE_M) q.values.slices = fg_value_slices(q.values, cdiv(q.M, q.bm) * cdiv(q.N, FG_BN), FG_THREADS * (q.split ? q.groups : 1));
-    FgParams p = fg_params(q);
+    const FgParams p = fg_params(q);
+    FgCarried carried = {};
     const int splits = (int)cdiv(q.K, p.kchunk);
     const int64_t tiles = cdiv(q.M, q.bm) * cdiv(q.N, FG_BN);
     const int groups = q.split ? q.groups : 1;
-    if (BSRC == FG_NOISE_I) p.sum_slices = (int)cdiv(cdiv(q.sum.blocks, groups), tiles);
+    if (BSRC == FG_NOISE_I) carried.sum_slices = (int)cdiv(cdiv(q.sum.blocks, groups), tiles);
     if (fg_carries_bias(ASRC, BSRC) && q.bias_grad.blocks) {
         const BiasGrad &g = q.bias_grad;
-        if (bias_direct(g.rows, g.n, g.bf16 ? 2 : 4, g.k, num_cus, FG_THREADS * groups)) p.bias_slices = (int)cdiv(g.blocks, tiles);
-        else if (int rc = bias_direct_launch(g, s)) return rc;   // too few threads to a block
+        if (q.split && bias_direct(g.rows, g.n, g.bf16 ? 2 : 4, g.k, num_cus, FG_THREADS * groups)) carried.bias_slices = (int)cdiv(g.blocks, tiles);
+        else if (int rc = bias_direct_launch(g, s)) return rc;   // too few threads to a block, or fp32 matrix instructions (rdb_set_f32_split), whose kernels carry nothing
+    }
+    const int more = carried.sum_slices + carried.bias_slices;
+    if (more) {
+        static_cast<FgParams &>(carried) = p;
+        carried.sum = q.sum;
+        carried.bias_grad = q.bias_grad;
     }
     const bool vec = fg_vec(q, ASRC, BSRC);
     const bool a16 = (ASRC == FG_KCONT || ASRC == FG_MCONT) && q.a_es == 2, b16 = (BSRC == FG_KCONT || BSRC == FG_MCONT) && q.b_es == 2;
     if (q.split && ((a16 && b16) ? !Groups::a16_b16 : a16 ? !Groups::a16_b32 : b16 && !Groups::a32_b16)) return RDB_E_UNSUPPORTED;
-    const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)(splits + (BSRC == FG_NOISE_M ? q.values.slices : 0) + p.sum_slices + p.bias_slices));
+    const dim3 grid((unsigned)cdiv(q.M, q.bm), (unsigned)cdiv(q.N, FG_BN), (unsigned)(splits + (BSRC == FG_NOISE_M ? q.values.slices : 0) + more));
     auto run = [&](auto epi_) {
         constexpr int EPI = decltype(epi_)::value;
         if (q.bm == 128 && q.groups == 2) FG_LAUNCH_GROUPS(128, 2, EPI);

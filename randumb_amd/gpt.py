@@ -6,7 +6,8 @@ block are qkv (d -> 3d), proj (d -> d), fc (d -> 4d) and mlp-proj (4d -> d), all
 dimension k and seeds taken in layer order from one generator (0..47 for 12 layers); attention is plain causal
 scaled-dot-product attention (the reference's FlexAttention document mask needs a tracing compiler); the token embedding
 and the language-model head are ordinary dense layers unless the configuration asks for the reference's random-backed ones
-(modded-nanogpt/gpt_models.py:303, 310).  This file wires layers: the linears' kernels are reached through SillyLinear.  The rest of a
+(modded-nanogpt/gpt_models.py:303, 310).  This file wires layers: the linears' kernels are reached through SillyLinear, but for an MLP of two
+plain layers, whose squared ReLU is formed and differentiated in the kernels that store their rows (RT_MLP).  The rest of a
 block (normalisation, rotary attention with a head dimension of 64, squared ReLU, the loss) is stock PyTorch, except in bf16 on the
 GPU, run eagerly: chains of stock operators took 6 times what the linears' kernels take there, most of it in passes over memory
 that the fused ones do not make.

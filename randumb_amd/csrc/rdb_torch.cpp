@@ -503,8 +503,8 @@ Tensor relu_squared_with_graph(const Tensor &x, const Tensor &dy);
 // The forward pass keeps z = x.N^T (and, in bf16, the transposed coefficients) for the backward pass, which needs nothing else
 // of x; with the fused random bias its full-rank share is added on top in both directions and x is saved as well.
 // square: where relu(y)^2 is left beside y, for a layer of that input (or NULL).
-// squared: the layer's input is relu(x)^2, formed here unless `formed` is that, which nothing keeps, and its gradient goes through that on its way to memory (8192 tokens x 3072 -> 768, k = 256:
-// backward and a pass over its dx 62.8 us, 47.7 so).
+// squared: the layer's input is relu(x)^2 of an x that wants a gradient, formed here unless `formed` is that, which nothing keeps, and its gradient goes through that on its way to
+// memory (8192 tokens x 3072 -> 768, k = 256: backward and a pass over its dx 62.8 us, 47.7 so); x is saved for it.
 class ProjectedLinear : public Function<ProjectedLinear> {
   public:
     static Tensor forward(AutogradContext *ctx, const Tensor &x0, const Tensor &coefs, const OptTensor &bias, const OptTensor &bias_scale, int64_t bias_seed,
@@ -1234,8 +1234,8 @@ PyObject *py_linear_projected(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
 }
 
-// relu_square_linear(x, coefs, in_f, out_f, seed): linear_projected of relu(x)^2, for a backward pass to come (None without one, or where
-// ops.linear runs another form)
+// relu_square_linear(x, coefs, in_f, out_f, seed): linear_projected of relu(x)^2, for a gradient of x to come; None without one: the node would save nothing of the
+// backward pass, and keep x for it
 PyObject *py_relu_square_linear(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
     return guarded([&]() -> PyObject * {
@@ -1244,14 +1244,14 @@ PyObject *py_relu_square_linear(PyObject *, PyObject *const *a, Py_ssize_t n)
         const Layer l{int_arg(a[2]), int_arg(a[3]), int_arg(a[2]), 1, seed_arg(a[4])};
         same_device("linear_fwd", x, {&c});
         check_sizes("linear_fwd", x, c, l, OptTensor(), Bias{});
-        if (!past_dispatcher({&x, &c}) || !at::GradMode::is_enabled() || !(x.requires_grad() || c.requires_grad())) Py_RETURN_NONE;
+        if (!past_dispatcher({&x, &c}) || !at::GradMode::is_enabled() || !x.requires_grad()) Py_RETURN_NONE;
         need_bf16("relu_square_linear", x);
         return THPVariable_Wrap(ProjectedLinear::apply(x, c, OptTensor(), OptTensor(), -1, OptTensor(), l, true, (const Tensor *)nullptr, (Tensor *)nullptr));
     });
 }
 
 // squared_relu_mlp(x, coefs 1, coefs 2, in_f, hidden, out_f, seed 1, seed 2): linear_projected, relu(.)^2 and linear_projected, each a node of its own but for the
-// activation, which is the second one's and leaves the first one's kernel beside its input; None as relu_square_linear
+// activation, which is the second one's and leaves the first one's kernel beside its input; None without a backward pass to come
 PyObject *py_squared_relu_mlp(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
     return guarded([&]() -> PyObject * {

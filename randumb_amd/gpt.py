@@ -177,7 +177,8 @@ class RT_MLP(nn.Module):
 
     def _proj_of_relu_square(self, h: torch.Tensor, ext):
         """Both in one autograd node, whose backward pass needs no pass over memory of its own for the activation; None where the layer is
-        more than its forward, or no backward pass is to come."""
+        more than its forward, or h wants no gradient.  For MLPs whose c_fc is called for itself: it has a hook, a bias, another class.  Forward and backward of
+        8192 tokens, 768 -> 3072 -> 768, c_fc with a hook: k = 256 189 -> 173 us, 128 172 -> 154; 1024 -> 4096 -> 1024, k = 256 254 -> 220; 2048 tokens even."""
         p = self.c_proj
         q = _plain_layer(p, h) if torch.is_grad_enabled() else None
         in_f, out_f = p.in_features, p.out_features

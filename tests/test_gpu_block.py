@@ -355,6 +355,40 @@ def test_squared_relu_in_the_projections_node(dim, k, tokens, kind):
     assert not torch.is_grad_enabled() or kind == "frozen input" or "ReluSquare" not in str(node(y)) and "ReluSquare" in str([node(y2)] + [f[0] for f in node(y2).next_functions])
 
 
+@pytest.mark.parametrize("first_half", ["trained", "frozen", "frozen, its input not"])
+@pytest.mark.parametrize("dim,k,tokens", [(64, 64, 40), (192, 136, 700)])
+def test_what_the_squared_relu_keeps(dim, k, tokens, first_half):
+    """From the forward to the backward pass: as many bytes as the layers and the activation keep where each is called for itself, none of them the
+    activation's input where that has no gradient."""
+    from randumb_amd.gpt import RT_GPTConfig, RT_MLP
+
+    print(f"case what the squared ReLU keeps dim={dim} k={k}, first half {first_half}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(dim)
+    with torch.device("cuda"):
+        mlp = RT_MLP(dim, RT_GPTConfig(int_dim_gen=iter([k, k]), seed_gen=iter([3, 4]))).bfloat16()
+    mlp.c_fc.weight_coef.requires_grad_(first_half == "trained")
+    x, dy = bf16(g, tokens, dim).requires_grad_(first_half != "frozen"), bf16(g, tokens, dim)
+    kept = []
+
+    def run():
+        kept.append([])
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: (kept[-1].append(t), t)[1], lambda t: t):
+            y = mlp(x)
+        torch.autograd.grad(y, mlp.c_proj.weight_coef, dy)
+
+    run()
+    handles = [mlp.c_fc.register_forward_hook(lambda m, args, out: None)]
+    run()
+    handles.append(mlp.c_proj.register_forward_hook(lambda m, args, out: None))
+    run()
+    bytes_of = [sum(t.untyped_storage().nbytes() for t in run_kept) for run_kept in kept]
+    assert bytes_of == bytes_of[-1:] * 3, bytes_of
+    hidden = [[t.shape[-1] for t in run_kept].count(4 * dim) for run_kept in kept]
+    assert hidden == [0 if first_half == "frozen" else 1] * 3, hidden
+    for h in handles:
+        h.remove()
+
+
 # one position, one row; fewer positions than waves; a last block of one row; rows of more than a wave's share (65, all, and half of the positions); columns of one
 # piece, of a part of one and of several
 @pytest.mark.parametrize("positions,vocab,dim,hot", [(1, 1, 8, 0), (7, 129, 64, 0), (600, 65, 520, 0), (1000, 64, 768, 65), (8192, 5030, 768, 4096), (3000, 40, 1032, 3000),

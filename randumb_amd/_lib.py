@@ -163,7 +163,7 @@ def load() -> ctypes.CDLL:
             "(hipcc, --offload-arch=gfx950). randumb_amd has no other compute path."
         )
     L = ctypes.CDLL(SO_PATH)
-    i64, u32, vp, ci = ctypes.c_int64, ctypes.c_uint32, ctypes.c_void_p, ctypes.c_int
+    i64, u32, vp, ci, f32 = ctypes.c_int64, ctypes.c_uint32, ctypes.c_void_p, ctypes.c_int, ctypes.c_float
     L.rdb_abi_version.restype = ci
     L.rdb_abi_version.argtypes = []
     # a library built from other sources may export the same names with other argument lists: calling those with this
@@ -215,7 +215,7 @@ def load() -> ctypes.CDLL:
     L.rdb_linear_rbias_fwd.argtypes = [vp, i64, vp, i64, vp, dp, vp]
     L.rdb_linear_rbias_fwd_ws.argtypes = [vp, i64, vp, i64, vp, dp, vp, i64, vp]
     L.rdb_linear_bwd_projected_rbias.argtypes = [vp, i64, vp, ci, vp, ci, vp, i64, vp, vp, i64, vp, vp, dp, vp, i64, vp]
-    L.rdb_linear_project_fwd_rbias.argtypes = [vp, i64, vp, i64, vp, vp, vp, vp, dp, vp, i64, vp]
+    L.rdb_linear_project_fwd_rbias.argtypes = [vp, i64, vp, vp, i64, vp, vp, vp, dp, vp, i64, vp]
     L.rdb_linear_rbias_bwd.argtypes = [vp, i64, vp, vp, i64, vp, i64, vp, dp, vp, i64, vp]
     L.rdb_linear_rbias_bwd_to.argtypes = [vp, i64, vp, ci, vp, i64, vp, i64, vp, dp, vp, i64, vp]
     L.rdb_linear_projection_bytes.argtypes = [dp]
@@ -273,11 +273,22 @@ def load() -> ctypes.CDLL:
     L.rdb_selftest_sync_giveup.restype = ci
     L.rdb_selftest_hasty_wait.argtypes = [vp, i64, vp, vp, i64, vp, dp, ci, vp]
     L.rdb_selftest_hasty_wait.restype = ci
+    L.rdb_rms_norm_fwd.argtypes = [vp, vp, vp, vp, vp, i64, i64, f32, vp]
+    L.rdb_rms_norm_bwd.argtypes = [vp, vp, vp, vp, vp, i64, i64, vp]
+    L.rdb_relu_square.argtypes = [vp, vp, vp, i64, vp]
+    L.rdb_cross_entropy_fwd.argtypes = [vp, vp, vp, vp, i64, i64, i64, vp]
+    L.rdb_cross_entropy_bwd.argtypes = [vp, vp, vp, vp, vp, i64, i64, i64, vp]
+    L.rdb_causal_attention_scratch_floats.argtypes = [i64, i64, i64]
+    L.rdb_causal_attention_scratch_floats.restype = i64
+    L.rdb_causal_attention_fwd.argtypes = [vp, vp, vp, vp, vp, vp, ci, i64, i64, i64, f32, vp]
+    L.rdb_causal_attention_bwd.argtypes = [vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, f32, vp]
     for name in ("rdb_sq5_fill_2d", "rdb_sq5_fill_1d", "rdb_materialize_fwd", "rdb_materialize_bwd", "rdb_scale_bias_bwd",
                  "rdb_embed_fwd", "rdb_embed_bwd", "rdb_linear_fwd", "rdb_linear_bwd_dx", "rdb_linear_bwd_dx_dscale", "rdb_linear_rbias_fwd",
                  "rdb_linear_rbias_fwd_ws", "rdb_linear_project_fwd_rbias", "rdb_linear_bwd_projected_rbias", "rdb_linear_rbias_bwd", "rdb_linear_rbias_bwd_to", "rdb_linear_bwd_dcoef",
                  "rdb_linear_project", "rdb_linear_project_fwd", "rdb_linear_fwd_projected", "rdb_linear_bwd_dcoef_projected",
-                 "rdb_linear_bwd_projected", "rdb_linear_bwd_projected_to", "rdb_linear_bwd_projected_part"):
+                 "rdb_linear_bwd_projected", "rdb_linear_bwd_projected_to", "rdb_linear_bwd_projected_part",
+                 "rdb_rms_norm_fwd", "rdb_rms_norm_bwd", "rdb_relu_square", "rdb_cross_entropy_fwd", "rdb_cross_entropy_bwd",
+                 "rdb_causal_attention_fwd", "rdb_causal_attention_bwd"):
         getattr(L, name).restype = ci
     _lib = L
     return L

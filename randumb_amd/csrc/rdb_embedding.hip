@@ -4,7 +4,8 @@
 // Its eight waves take an eighth of the positions each, so that their lists, one behind the other, are in the order of the positions: fixed sums, in fp32,
 // rounded once.  The block's lists together are mostly shorter than a wave, and then lie in one register.  A row of up to 64 positions is one wave's; one of more,
 // a chain of that many loads, is all waves', each the positions of its own list, sixteen rows of dy in flight.  us, kernel alone, and the stock call with its launches:
-// 50304 x 768, 8192 positions 27, 112; 1024 24, 77; 16384 48, 146; half of 8192 at one row 195, 204; all of them 207, 304; 50304 x 256, 64 positions 18, 26.
+// 50304 x 768, 8192 positions 27, 112; 1024 24, 77; 16384 31, 146 (48 with one block to a compute unit); half of 8192 at one row 181, 204; all of them 206, 304; 50304 x 256,
+// 64 positions 19, 26.
 #include "rdb_common.hpp"
 #include <algorithm>
 #include <type_traits>
@@ -13,15 +14,17 @@ namespace rdb {
 
 int num_compute_units();   // rdb_error.hip
 constexpr int EG_ROW_BITS = 7, EG_ROWS = 1 << EG_ROW_BITS, EG_WAVES = 8, EG_THREADS = EG_WAVES * 64, EG_PIECE = 512, EG_LIGHT = 64, EG_AHEAD = 8;
-constexpr int64_t EG_POSITIONS = 16384;   // as many as the lists have room for in LDS, 4 bytes each
+constexpr int64_t EG_POSITIONS = 16384;   // as many as the lists of two blocks have room for in a compute unit's LDS, 4 bytes each
+constexpr int64_t EG_SUMS_BYTES = (EG_WAVES - 1) * EG_PIECE * (int64_t)sizeof(float);
+static_assert(2 * (EG_SUMS_BYTES + EG_POSITIONS * 4 + (EG_ROWS + EG_WAVES) * 4) <= 160 * 1024, "two blocks to a compute unit");
 
 template <typename I> __global__ __launch_bounds__(EG_THREADS) void embedding_grad_kernel(bf16_t *__restrict__ dw, const I *__restrict__ idx, const bf16_t *__restrict__ dy,
                                                                                           int positions, int each, int64_t vocab, int dim, int block_rows)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int hist[EG_ROWS], count[EG_WAVES];
-    float *const sums = reinterpret_cast<float *>(smem);                              // [EG_WAVES][EG_PIECE]
-    uint32_t *const lists = reinterpret_cast<uint32_t *>(sums + EG_WAVES * EG_PIECE);   // [EG_WAVES][each]: position << EG_ROW_BITS | row of the block
+    float *const sums = reinterpret_cast<float *>(smem);                                    // [EG_WAVES - 1][EG_PIECE]: those of wave 0 stay in its registers
+    uint32_t *const lists = reinterpret_cast<uint32_t *>(sums + (EG_WAVES - 1) * EG_PIECE);   // [EG_WAVES][each]: position << EG_ROW_BITS | row of the block
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t row0 = (int64_t)blockIdx.x * block_rows;
     if (threadIdx.x < EG_ROWS) hist[threadIdx.x] = 0;
@@ -118,16 +121,16 @@ template <typename I> __global__ __launch_bounds__(EG_THREADS) void embedding_gr
         for (int col = lane * 8; col < (dim + EG_PIECE - 1) / EG_PIECE * EG_PIECE; col += EG_PIECE) {
             clear();
             add(std::integral_constant<int, 16>{}, wave, r, col);
+            if (wave) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) sums[wave * EG_PIECE + j * 64 + lane] = acc[j];
+                for (int j = 0; j < 8; ++j) sums[(wave - 1) * EG_PIECE + j * 64 + lane] = acc[j];
+            }
             __syncthreads();
             if (wave == 0) {
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    acc[j] = sums[j * 64 + lane];
+                for (int j = 0; j < 8; ++j)
 #pragma unroll
-                    for (int w = 1; w < EG_WAVES; ++w) acc[j] += sums[w * EG_PIECE + j * 64 + lane];
-                }
+                    for (int w = 1; w < EG_WAVES; ++w) acc[j] += sums[(w - 1) * EG_PIECE + j * 64 + lane];
                 store(r, col);
             }
             __syncthreads();
@@ -155,7 +158,7 @@ extern "C" int rdb_embedding_bwd(void *dweight, const void *idx, int idx_bytes, 
         return set_error(RDB_E_ALIGN, "rdb_embedding_bwd: dweight and dy must be 16-byte aligned");
     const int each = (int)((positions + EG_WAVES - 1) / EG_WAVES);
     const int64_t cus = num_compute_units(), block_rows = std::min<int64_t>(EG_ROWS, std::max<int64_t>(8, (vocab + 2 * cus - 1) / (2 * cus)));
-    const size_t smem = (size_t)EG_WAVES * EG_PIECE * sizeof(float) + (size_t)EG_WAVES * each * sizeof(uint32_t);
+    const size_t smem = (size_t)EG_SUMS_BYTES + (size_t)EG_WAVES * each * sizeof(uint32_t);
     auto launch = [&](auto zero) {
         typedef decltype(zero) I;
         if (int rl = reserve_lds(reinterpret_cast<const void *>(embedding_grad_kernel<I>), smem, "embedding_grad_kernel")) return rl;

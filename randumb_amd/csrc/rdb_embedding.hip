@@ -142,16 +142,32 @@ template <typename I> __global__ __launch_bounds__(EG_THREADS) void embedding_gr
 
 using namespace rdb;
 
+// what one launch can do: the grid's threads stay below 2^32
+static bool embedding_fits(int64_t positions, int64_t vocab, int64_t dim)
+{
+    return positions > 0 && positions <= EG_POSITIONS && vocab > 0 && vocab <= (1ll << 29) && dim > 0 && dim % 8 == 0 && dim <= (1 << 20);
+}
+
+// Where that is the faster way.  Every block looks through all indices, so a long table costs rounds of blocks, some 12 us each, however few its columns; the stock call costs 25 us with few
+// positions, 55 at 1024, 80 to 110 from there on, and the clearing of the table.  us, this one and the stock one, on either side of each line (256 compute units: a round is 65536 rows):
+//   one round, with few positions and a long or wide table, which is cleared faster than its rows are written one by one: 64 positions, 50304 x 768 22.9, 26.4; 65536 x 768 28.3, 27.7;
+//   50304 x 2048 37.9, 33.1; 512 positions 39.4, 61.4
+//   rounds against positions: two, x 64 columns: 512 positions 38.1, 32.2; 1024 38.0, 57.8; three: 1024 55.1, 59.8; four: 1024 72.3, 70.6; 2048 73.0, 132
+//   rounds, 4096 positions: four, x 256 74, 95; five 91, 97; seven 112, 100; eight 142, 98; x 768, whose writing takes longer than the indices: eight 187, 198; thirteen 265, 261; a million rows x 8:
+//   246, 99
 extern "C" int rdb_embedding_bwd_takes(int64_t positions, int64_t vocab, int64_t dim)
 {
-    return positions > 0 && positions <= EG_POSITIONS && vocab > 0 && vocab <= (1ll << 31) && dim > 0 && dim % 8 == 0 && dim <= (1 << 20) ? 1 : 0;
+    if (!embedding_fits(positions, vocab, dim)) return 0;
+    const int64_t round = 2 * (int64_t)EG_ROWS * num_compute_units(), rounds = (vocab + round - 1) / round;
+    if (rounds == 1) return positions >= 512 || vocab * dim <= (3 << 24) ? 1 : 0;
+    return rounds <= (dim >= 768 ? 8 : 4) && positions >= 512 * rounds ? 1 : 0;
 }
 
 extern "C" int rdb_embedding_bwd(void *dweight, const void *idx, int idx_bytes, const void *dy, int64_t positions, int64_t vocab, int64_t dim, void *stream)
 {
     if (positions < 0 || vocab < 0 || dim < 0) return set_error(RDB_E_SHAPE, "rdb_embedding_bwd: negative size");
-    if (!rdb_embedding_bwd_takes(positions, vocab, dim))
-        return set_error(RDB_E_UNSUPPORTED, "rdb_embedding_bwd: 1 to %lld positions and a multiple of 8 columns", (long long)EG_POSITIONS);
+    if (!embedding_fits(positions, vocab, dim))
+        return set_error(RDB_E_UNSUPPORTED, "rdb_embedding_bwd: 1 to %lld positions, up to 2^29 rows and a multiple of 8 columns", (long long)EG_POSITIONS);
     if (!dweight || !idx || !dy) return set_error(RDB_E_NULL, "rdb_embedding_bwd: dweight, idx or dy is NULL");
     if (idx_bytes != 4 && idx_bytes != 8) return set_error(RDB_E_DTYPE, "rdb_embedding_bwd: indices of 4 or 8 bytes");
     if (((uintptr_t)dweight & 15) || ((uintptr_t)dy & 15) || ((uintptr_t)idx & (uintptr_t)(idx_bytes - 1)))

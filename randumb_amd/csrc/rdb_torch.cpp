@@ -1368,7 +1368,7 @@ PyObject *py_relu_square(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
 }
 
-// embedding(weight, idx): rows of a dense bf16 table; None without a backward pass to come, or for sizes that its kernel does not take
+// embedding(weight, idx): rows of a dense bf16 table; None without a backward pass to come, or for sizes that the stock operator is faster at
 PyObject *py_embedding(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
     return guarded([&]() -> PyObject * {

@@ -410,6 +410,17 @@ def test_gradient_of_a_dense_table(ext, positions, vocab, dim, hot, dtype):
     assert torch.equal(torch.autograd.grad(ext.embedding(w, idx), w, dy)[0], got)
 
 
+# tables of several rounds of blocks, the last one of one row; a row of many positions among them
+@pytest.mark.parametrize("positions,vocab,dim,hot", [(1024, 65537, 8, 100), (2048, 262144, 24, 1000), (4096, 270000, 768, 0)])
+def test_gradient_of_a_long_table(ext, positions, vocab, dim, hot):
+    test_gradient_of_a_dense_table(ext, positions, vocab, dim, hot, torch.int64)
+
+
+def test_long_tables_are_left_to_the_stock_operator(ext):
+    w, idx = torch.zeros(300000, 8, device="cuda", dtype=torch.bfloat16, requires_grad=True), torch.zeros(4096, dtype=torch.int64, device="cuda")
+    assert ext.embedding(w, idx) is None and ext.embedding(w[:131072], idx) is not None and ext.embedding(w[:131072], idx[:1000]) is None
+
+
 def test_dense_tables_that_the_kernel_leaves(ext):
     w, many = torch.zeros(10, 64, device="cuda", dtype=torch.bfloat16, requires_grad=True), torch.zeros(16385, dtype=torch.int64, device="cuda")
     assert ext.embedding(w, many) is None and ext.embedding(w, many[:0]) is None and ext.embedding(w.detach(), many[:5]) is None

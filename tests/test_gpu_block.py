@@ -333,11 +333,12 @@ def test_squared_relu_in_the_projections_node(dim, k, tokens, kind):
                 y = mlp(x)
         else:
             y = mlp(x)
-        if kind == "second derivative":   # of c_proj's input gradient behind the activation, in what feeds the activation
+        if kind == "second derivative":   # the layers have none: each of the first derivatives in what it depends on
             first = torch.autograd.grad(y, leaves, dy, create_graph=True)
-            with pytest.raises(RuntimeError, match="no second derivative"):
-                torch.autograd.grad(first[2].float().sum(), leaves[2], retain_graph=True, allow_unused=True)
-                torch.autograd.grad(first[0].float().square().sum(), x)
+            for of, leaf in ((0, 0), (0, 1), (0, 2), (1, 0), (1, 2), (2, 0), (2, 1)):
+                with pytest.raises(RuntimeError, match="no second derivative"):
+                    torch.autograd.grad(first[of].float().square().sum(), leaves[leaf], retain_graph=True)
+            assert torch.autograd.grad(first[2].float().square().sum(), leaves[2], retain_graph=True, allow_unused=True) == (None,)   # dC = dy^T . z
             return y, [f.detach() for f in first]
         return y, torch.autograd.grad(y, leaves, dy)
 
@@ -353,6 +354,29 @@ def test_squared_relu_in_the_projections_node(dim, k, tokens, kind):
     assert len(seen) == 2 and torch.equal(y, y2) and all(torch.equal(a, b) for a, b in zip(grads, grads2))
     node = lambda t: t.grad_fn.next_functions[0][0].next_functions[0][0]
     assert not torch.is_grad_enabled() or kind == "frozen input" or "ReluSquare" not in str(node(y)) and "ReluSquare" in str([node(y2)] + [f[0] for f in node(y2).next_functions])
+
+
+@pytest.mark.parametrize("dim,k,tokens", [(64, 64, 40), (192, 136, 700), (72, 64, 520)])
+def test_second_derivative_of_the_squared_relu(ext, dim, k, tokens):
+    """In the projection's node, whose layer has none: dx under create_graph depends on what feeds the activation as the stock operators' does, and on the
+    coefficients by what raises."""
+    from randumb_amd import ops
+
+    print(f"case second derivative of the squared ReLU dim={dim} k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(dim)
+    h, dy, v, c = bf16(g, tokens, 4 * dim).requires_grad_(), bf16(g, tokens, dim), bf16(g, tokens, 4 * dim), bf16(g, dim, k)
+    y = ext.relu_square_linear(h, c, 4 * dim, dim, 3)
+    dx, = torch.autograd.grad(y, h, dy, create_graph=True)
+    got, = torch.autograd.grad(dx, h, v)
+    a = F.relu(h.detach()).square().requires_grad_()
+    behind, = torch.autograd.grad(ops.linear(a, c, 4 * dim, dim, 4 * dim, 1, 3, None, None), a, dy)
+    want_dx, want = behind.double() * 2 * F.relu(h).detach().double(), v.double() * behind.double() * 2 * (h > 0)
+    for x, w in ((dx, want_dx), (got, want)):   # a few products of bf16 values, each rounded
+        assert bool(((x.detach().double() - w).abs() <= 2.0**-6 * w.abs()).all()) and float(w.abs().sum()) > 0
+    c.requires_grad_()
+    dx, = torch.autograd.grad(ext.relu_square_linear(h, c, 4 * dim, dim, 3), h, dy, create_graph=True)
+    with pytest.raises(RuntimeError, match="no second derivative"):
+        torch.autograd.grad(dx, c, v)
 
 
 @pytest.mark.parametrize("first_half", ["trained", "frozen", "frozen, its input not"])

@@ -488,7 +488,7 @@ template <typename E, int TC, int WAVES> __global__ __launch_bounds__(WAVES * 64
 // an expanding block reads eight at a time: 1 x 4096 -> 4096, k = 16: chunks of 128, 256, 512, 1024: 8.9, 8.0, 8.2, 10.9 us).
 // waves: a wave hashes 32 contraction values for its 16 coefficients, which a SIMD with a single wave does at half its rate, and the blocks are fewer than the chip holds; so
 // a chunk of 512 is 16 waves, or 8 where an expanding block is as large (more have no registers for that; k > 256: four).  us per call, four waves -> so: 16 x 4096 -> 11008, k = 256,
-// bf16 11.4 -> 11.0; 64 tokens 18.6 -> 17.3; 8 x 8192 -> 8192, k = 512 21.9 -> 19.9; in one launch: 1 x 4096 -> 4096, k = 16, fp32 8.9 -> 8.1; 4 x 2000 -> 5000, k = 100 9.5 -> 8.7;
+// bf16 11.3 -> 10.7 to 11.2; 64 tokens 18.6 -> 17.3; 8 x 8192 -> 8192, k = 512 21.9 -> 19.9; in one launch: 1 x 4096 -> 4096, k = 16, fp32 8.9 -> 8.1; 4 x 2000 -> 5000, k = 100 9.5 -> 8.7;
 // 16 x 4096 -> 4096, k = 128 11.1 -> 10.6.  (Chunks of 1024 and 2048 in 16 waves, half and a quarter of the partial sums: 11.8 and 15.1 for the first.  Expanding blocks of eight waves in
 // a launch of their own: 64 tokens 20.7.)  The number depends on the layer alone, so that the same sums come out in one launch and in two.
 // te: tiles of an expanding block.  Finer is sooner ready while the blocks run side by side, two (of k > 128: one) to a compute unit: 64 x

@@ -699,7 +699,7 @@ static int product_room(int64_t M, int64_t N, int64_t K, int num_cus) { return f
 static bool product_ok(int64_t M, int64_t N, int64_t K) { return M > 0 && N > 0 && K > 0 && M * N < (1ll << 29) && K < (1 << 30); }
 
 // The products of a vector-coef layer's backward pass, dx = dy . W and dW = dy^T . x, side by side in one launch where both are wanted; what is left to
-// add up is left to a launch that comes anyway: dx's ranges (dx_sum, blocks 0: there are none), and dW's, as partial matrices (dw).
+// add up is left to a launch that comes anyway: dx's ranges (dx_sum, blocks 0: there are none), and up to VECTOR_DW_PARTS of dW's, as partial matrices (dw).
 static bool vector_products_ok(int64_t tokens, int64_t in_f, int64_t out_f)
 {
     return product_ok(tokens, in_f, out_f) && product_ok(out_f, in_f, tokens) && tokens * out_f < (1ll << 29) && tokens * in_f < (1ll << 29) && f32_split_mode();
@@ -707,9 +707,11 @@ static bool vector_products_ok(int64_t tokens, int64_t in_f, int64_t out_f)
 // dW's ranges: its partial matrices are added up where dW is contracted with the noise, which is the vector ALU's, so they cost memory traffic and its power: at most 16 MB
 // of them.  Vector-coef steps, us, with one, two, four, eight ranges at most: 1024 tokens x 512 -> 1024, k = 200 130, 118, 117, 118; 1500 x 300 -> 3000, k = 60 146,
 // 147, 130, 131; 2048 x 1024 -> 1024, k = 256 256, 245, 245, 244; 1024 x 768 -> 3072, k = 256, kept up for a second: 464, 475, 475, 477.
+// Many tokens of a small layer are more ranges than the contraction holds on the way (VECTOR_DW_PARTS): they and dx's are added up by a launch of their own then.  Eight at most
+// and so, us: 30138 x 111 -> 331, k = 111 217, 131 (eight launches 145); 13811 x 135 -> 211, k = 52 96, 80 (85); 9080 x 280 -> 560, k = 18 130, 109 (118).
 static int vector_dw_room(int64_t tokens, int64_t in_f, int64_t out_f, int num_cus)
 {
-    const int64_t most = std::max<int64_t>(1, std::min<int64_t>(VECTOR_DW_PARTS, (16 << 20) / (out_f * in_f * 4)));
+    const int64_t most = std::max<int64_t>(1, (16 << 20) / (out_f * in_f * 4));
     return (int)std::min<int64_t>(product_room(out_f, in_f, tokens, num_cus), most);
 }
 // scratch: dx's partial matrices and dW's (or dW); 0: not taken
@@ -717,7 +719,8 @@ int64_t vector_products_workspace(int64_t tokens, int64_t in_f, int64_t out_f, b
 {
     if (!vector_products_ok(tokens, in_f, out_f)) return 0;
     const int num_cus = num_compute_units(), r = want_dx ? product_room(tokens, in_f, out_f, num_cus) : 1;
-    return (r > 1 ? r : 0) * up256(tokens * in_f * 4) + vector_dw_room(tokens, in_f, out_f, num_cus) * up256(out_f * in_f * 4);
+    const int dw = vector_dw_room(tokens, in_f, out_f, num_cus);
+    return (r > 1 ? r : 0) * up256(tokens * in_f * 4) + (dw > VECTOR_DW_PARTS ? dw + 1 : dw) * up256(out_f * in_f * 4);
 }
 int vector_products(float *dx, const float *dy, int64_t lddy, const float *x, int64_t ldx, const float *W, int64_t tokens, int64_t in_f, int64_t out_f,
                     void *workspace, FgSum *dx_sum, VectorDW *dw, hipStream_t s)
@@ -729,6 +732,16 @@ int vector_products(float *dx, const float *dy, int64_t lddy, const float *x, in
     FgProduct qx = {dy, lddy, (tokens - 1) * lddy + out_f, W, in_f, out_f * in_f, dx, in_f, nullptr, tokens, in_f, out_f, 0, 0, 0, 0, 0u};
     FgProduct qw = {dy, lddy, (tokens - 1) * lddy + out_f, x, ldx, (tokens - 1) * ldx + in_f, dw_part, in_f, nullptr, out_f, in_f, tokens, 0, 0, 0, 0, 0u};
     *dx_sum = {};
+    // what the contraction does not add up on its way
+    auto done = [&](int parts) {
+        *dw = {dw_part, dw_stride, parts};
+        if (parts <= VECTOR_DW_PARTS) return (int)RDB_OK;
+        float *const sum = dw_part + dw_room * dw_stride;
+        const int rc = fg_launch_sums(*dx_sum, fg_sum(sum, 0, dw_part, qw.M * qw.N, dw_stride, parts), s);
+        *dx_sum = {};
+        *dw = {sum, 0, 1};
+        return rc;
+    };
     auto ranges = [](FgProduct &q, int r, float *part, int64_t stride) {
         q.kchunk = r > 1 ? fg_chunk(q.K, r) : 0;
         if (r > 1) {
@@ -746,8 +759,7 @@ int vector_products(float *dx, const float *dy, int64_t lddy, const float *x, in
         const int rc = fg_launch_pair(tx, tw, s);
         if (rc != RDB_E_UNSUPPORTED) {
             *dx_sum = fg_sum(dx, 0, dx_part, qx.M * qx.N, dx_stride, plan.ranges[0]);
-            *dw = {dw_part, dw_stride, plan.ranges[1]};
-            return rc;
+            return rc ? rc : done(plan.ranges[1]);
         }
         const FgPlan px = fg_plan(qx.M, qx.N, qx.K, num_cus, room, FgGroups<FG_KCONT, FG_MCONT>::four);
         qx.bm = px.bm;
@@ -760,8 +772,8 @@ int vector_products(float *dx, const float *dy, int64_t lddy, const float *x, in
     qw.bm = pw.bm;
     qw.groups = pw.groups;
     ranges(qw, pw.ranges, dw_part, dw_stride);
-    *dw = {dw_part, dw_stride, pw.ranges};
-    return fg_launch<FG_MCONT, FG_MCONT>(qw, num_cus, s, "f32_gemm_kernel (dW = dy^T . x)");
+    const int rc = fg_launch<FG_MCONT, FG_MCONT>(qw, num_cus, s, "f32_gemm_kernel (dW = dy^T . x)");
+    return rc ? rc : done(pw.ranges);
 }
 
 }  // namespace rdb

@@ -94,7 +94,8 @@ def test_embedding(shape, dim, k):
     assert torch.equal(got, ops.embed_bwd(idx, dy, k, dim, 4))
 
 
-@pytest.mark.parametrize("tokens,in_f,out_f,k,bias_k", [(1, 1, 1, 1, 1), (33, 67, 130, 17, 0), (257, 300, 65, 40, 9), (700, 129, 1000, 256, 64), (1500, 300, 520, 100, 300)])
+@pytest.mark.parametrize("tokens,in_f,out_f,k,bias_k", [(1, 1, 1, 1, 1), (33, 67, 130, 17, 0), (257, 300, 65, 40, 9), (700, 129, 1000, 256, 64), (1500, 300, 520, 100, 300),
+                                                         (9000, 24, 40, 20, 5), (13001, 135, 67, 33, 0), (4100, 300, 129, 8, 70)])   # dW in more ranges than the contraction adds up
 def test_backward_pass_in_one_call(tokens, in_f, out_f, k, bias_k):
     """rdb_vector_linear_bwd against fp64 and against the calls it stands for: dx or not, a bias or not, rows that are slices."""
     from randumb_amd import _lib, hip

@@ -23,6 +23,14 @@ def _up(n, to=256):
 CASES = [(2048, 3072, 768, 256), (256, 8192, 1024, 512), (257, 8192, 1024, 32), (700, 4000, 256, 120), (492, 3184, 273, 118), (433, 3320, 96, 144)]
 
 
+@pytest.mark.parametrize("tokens,in_f,out_f", [(30138, 111, 331), (13811, 135, 211), (9080, 280, 560), (9000, 24, 40)])
+@pytest.mark.parametrize("dx", [0, 1])
+def test_many_tokens_of_a_small_vector_coef_layer(tokens, in_f, out_f, dx):
+    """The backward pass in one call has room for as many ranges of dW as the product alone, up to 16 MB: with eight at most its few tiles run on for most of the step."""
+    lib = _lib.load()
+    assert lib.rdb_vector_linear_bwd_workspace_bytes(tokens, in_f, out_f, 16, dx, 0) >= min(lib.rdb_product_f32_workspace_bytes(out_f, in_f, tokens), 16 << 20)
+
+
 @pytest.mark.parametrize("dtype", [_lib.RDB_BF16, _lib.RDB_F32])
 def test_nothing_but_what_the_backward_pass_reads(dtype):
     lib, rng = _lib.load(), random.Random(3)

@@ -709,9 +709,12 @@ static bool vector_products_ok(int64_t tokens, int64_t in_f, int64_t out_f)
 // 147, 130, 131; 2048 x 1024 -> 1024, k = 256 256, 245, 245, 244; 1024 x 768 -> 3072, k = 256, kept up for a second: 464, 475, 475, 477.
 // Many tokens of a small layer are more ranges than the contraction holds on the way (VECTOR_DW_PARTS): they and dx's are added up by a launch of their own then.  Eight at most
 // and so, us: 30138 x 111 -> 331, k = 111 217, 131 (eight launches 145); 13811 x 135 -> 211, k = 52 96, 80 (85); 9080 x 280 -> 560, k = 18 130, 109 (118).
-static int vector_dw_room(int64_t tokens, int64_t in_f, int64_t out_f, int num_cus)
+// Without dx beside it, whose tiles fill its last round, a long product of dW (2048 tokens and more) loses more to that round: 32 MB there.  No dx, 16 and 32 MB: 8192 x 768 -> 3072, k = 8
+// 539, 442 (469 as calls of their own); 19876 x 1288 -> 680, k = 4 539, 486 (501); 16384 x 1024 -> 1024, k = 8 384, 386; 1024 x 768 -> 3072, k = 256 447, 452; with dx 16384 x 1024 ->
+// 1024 514, 551, 32768 x 512 -> 512, k = 8 313, 334.
+static int vector_dw_room(int64_t tokens, int64_t in_f, int64_t out_f, bool dx, int num_cus)
 {
-    const int64_t most = std::max<int64_t>(1, (16 << 20) / (out_f * in_f * 4));
+    const int64_t most = std::max<int64_t>(1, (dx || tokens < 2048 ? 16 << 20 : 32 << 20) / (out_f * in_f * 4));
     return (int)std::min<int64_t>(product_room(out_f, in_f, tokens, num_cus), most);
 }
 // scratch: dx's partial matrices and dW's (or dW); 0: not taken
@@ -719,14 +722,14 @@ int64_t vector_products_workspace(int64_t tokens, int64_t in_f, int64_t out_f, b
 {
     if (!vector_products_ok(tokens, in_f, out_f)) return 0;
     const int num_cus = num_compute_units(), r = want_dx ? product_room(tokens, in_f, out_f, num_cus) : 1;
-    const int dw = vector_dw_room(tokens, in_f, out_f, num_cus);
+    const int dw = vector_dw_room(tokens, in_f, out_f, want_dx, num_cus);
     return (r > 1 ? r : 0) * up256(tokens * in_f * 4) + (dw > VECTOR_DW_PARTS ? dw + 1 : dw) * up256(out_f * in_f * 4);
 }
 int vector_products(float *dx, const float *dy, int64_t lddy, const float *x, int64_t ldx, const float *W, int64_t tokens, int64_t in_f, int64_t out_f,
                     void *workspace, FgSum *dx_sum, VectorDW *dw, hipStream_t s)
 {
     if (!vector_products_ok(tokens, in_f, out_f) || tokens * lddy >= (1ll << 29) || tokens * ldx >= (1ll << 29)) return RDB_E_UNSUPPORTED;
-    const int num_cus = num_compute_units(), room = dx ? product_room(tokens, in_f, out_f, num_cus) : 1, dw_room = vector_dw_room(tokens, in_f, out_f, num_cus);
+    const int num_cus = num_compute_units(), room = dx ? product_room(tokens, in_f, out_f, num_cus) : 1, dw_room = vector_dw_room(tokens, in_f, out_f, dx != nullptr, num_cus);
     const int64_t dx_stride = up256(tokens * in_f * 4) / 4, dw_stride = up256(out_f * in_f * 4) / 4;
     float *dx_part = static_cast<float *>(workspace), *dw_part = dx_part + (room > 1 ? room : 0) * dx_stride;
     FgProduct qx = {dy, lddy, (tokens - 1) * lddy + out_f, W, in_f, out_f * in_f, dx, in_f, nullptr, tokens, in_f, out_f, 0, 0, 0, 0, 0u};

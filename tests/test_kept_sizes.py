@@ -31,6 +31,13 @@ def test_many_tokens_of_a_small_vector_coef_layer(tokens, in_f, out_f, dx):
     assert lib.rdb_vector_linear_bwd_workspace_bytes(tokens, in_f, out_f, 16, dx, 0) >= min(lib.rdb_product_f32_workspace_bytes(out_f, in_f, tokens), 16 << 20)
 
 
+@pytest.mark.parametrize("tokens,in_f,out_f", [(8192, 768, 3072), (19876, 1288, 680)])
+def test_a_long_product_of_dw_alone_has_room_for_ranges(tokens, in_f, out_f):
+    """Without dx beside it there is nothing to fill its last round of tiles."""
+    lib = _lib.load()
+    assert lib.rdb_vector_linear_bwd_workspace_bytes(tokens, in_f, out_f, 8, 0, 0) >= min(lib.rdb_product_f32_workspace_bytes(out_f, in_f, tokens), 28 << 20)
+
+
 @pytest.mark.parametrize("dtype", [_lib.RDB_BF16, _lib.RDB_F32])
 def test_nothing_but_what_the_backward_pass_reads(dtype):
     lib, rng = _lib.load(), random.Random(3)

@@ -151,25 +151,30 @@ __device__ __forceinline__ void materialize_vec_block(const MatVecParams &p, flo
         p.out[n] = acc;
     }
 }
-template <bool GATHER, int LANES, bool SHORT> __global__ __launch_bounds__(NT) void materialize_vec_kernel(MatVecParams p)
+// TURNS: blocks take several turns (p.blocks of them in all); without, the kernel is one turn and nothing else: with the loop around it a short launch, which is all latency, takes
+// 0.4 us more (40 x 5 elements, k = 3: 2.2 -> 2.65 us)
+template <bool GATHER, int LANES, bool SHORT, bool TURNS>
+__device__ __forceinline__ void materialize_vec_turns(const MatVecParams &p, float *__restrict__ cs, unsigned first, unsigned blocks)
+{
+    bool one_factor = false;
+    if constexpr (TURNS) {
+        for (unsigned block = first; block < p.blocks; block += blocks)
+            materialize_vec_block<GATHER, LANES, SHORT>(p, cs, block, block == first || p.k > COEF_CHUNK, one_factor);
+    } else {
+        materialize_vec_block<GATHER, LANES, SHORT>(p, cs, first, true, one_factor);
+    }
+}
+template <bool GATHER, int LANES, bool SHORT, bool TURNS> __global__ __launch_bounds__(NT) void materialize_vec_kernel(MatVecParams p)
 {
     __shared__ __align__(16) float cs[COEF_CHUNK + MAT_UNROLL];   // reads run a turn ahead
-    bool one_factor = false;
-    for (unsigned block = blockIdx.x; block < p.blocks; block += gridDim.x)
-        materialize_vec_block<GATHER, LANES, SHORT>(p, cs, block, block == blockIdx.x || p.k > COEF_CHUNK, one_factor);
+    materialize_vec_turns<GATHER, LANES, SHORT, TURNS>(p, cs, blockIdx.x, TURNS ? gridDim.x : 0);
 }
 // A weight and its bias, contiguous both: the bias's blocks (16 lanes an element) first.
-template <int LANES, bool SHORT> __global__ __launch_bounds__(NT) void materialize_vec_pair_kernel(MatVecParams weight, MatVecParams bias, unsigned bias_blocks)
+template <int LANES, bool SHORT, bool TURNS> __global__ __launch_bounds__(NT) void materialize_vec_pair_kernel(MatVecParams weight, MatVecParams bias, unsigned bias_blocks)
 {
     __shared__ __align__(16) float cs[COEF_CHUNK + MAT_UNROLL];   // reads run a turn ahead
-    bool one_factor = false;
-    if (blockIdx.x < bias_blocks) {
-        materialize_vec_block<false, 16, false>(bias, cs, blockIdx.x, true, one_factor);
-        return;
-    }
-    const unsigned first = blockIdx.x - bias_blocks;
-    for (unsigned block = first; block < weight.blocks; block += gridDim.x - bias_blocks)
-        materialize_vec_block<false, LANES, SHORT>(weight, cs, block, block == first || weight.k > COEF_CHUNK, one_factor);
+    if (blockIdx.x < bias_blocks) materialize_vec_turns<false, 16, false, false>(bias, cs, blockIdx.x, 0);
+    else materialize_vec_turns<false, LANES, SHORT, TURNS>(weight, cs, blockIdx.x - bias_blocks, TURNS ? gridDim.x - bias_blocks : 0);
 }
 
 // Matrix-coef materialise, arbitrary view: one thread per output element (no sharing of noise between rows).
@@ -672,28 +677,34 @@ static void split_plan(int64_t Nw, int64_t k, int64_t *splits, int64_t *span)
 
 // lanes per element of a tensor of n values by k terms: as many as fill the chip's 8192 wave slots, of 1, 4, 16
 static int mat_lanes(int64_t n, int64_t k) { return k < 8 ? 1 : n <= (1 << 15) ? 16 : n <= (1 << 17) ? 4 : 1; }
+// as many blocks as are resident at once, which take the elements in turns: their coefficients are read once, and no unit is left with a block more
+// than others (blocks in turn -> so: 2.4 M elements, k = 256 173.7 -> 170.5 us; 0.8 M 65.6 -> 62.6; 1.5 M 113.6 -> 107.8; 2.9 M 215.0 -> 210.7; at most 0.5 M: even).  Several lanes to an
+// element: few elements.
+static unsigned mat_blocks(unsigned all, int lanes) { return lanes > 1 ? all : std::min(all, 8u * (unsigned)num_compute_units()); }
+template <class F> static void mat_variant(int lanes, int64_t k, bool turns, F &&f)
+{
+    auto with_terms = [&](auto lanes_, auto turns_) {
+        if (k <= MAT_SHORT) f(lanes_, std::true_type{}, turns_);
+        else f(lanes_, std::false_type{}, turns_);
+    };
+    if (lanes == 16) with_terms(std::integral_constant<int, 16>{}, std::false_type{});
+    else if (lanes == 4) with_terms(std::integral_constant<int, 4>{}, std::false_type{});
+    else if (turns) with_terms(std::integral_constant<int, 1>{}, std::true_type{});
+    else with_terms(std::integral_constant<int, 1>{}, std::false_type{});
+}
 static int launch_materialize_vec(float *out, const void *coef, int coef_dtype, int64_t k, int64_t Nw, int64_t Q, int64_t sP, int64_t sQ, uint32_t seed,
                                   const void *scale_bias, const int64_t *idx, hipStream_t s)
 {
     const int lanes = mat_lanes(Nw, k);
     const MatVecParams p = {out, coef, scale_bias, idx, k, Nw, Q, sP, sQ, coef_dtype, Nw < (1ll << 32) && Q < (1ll << 32), sQ == 1 && (sP == Q || Nw == Q), seed,
                             (unsigned)cdiv(Nw * lanes, NT)};
-    // as many blocks as are resident at once, which take the elements in turns: their coefficients are read once, and no unit is left with a block more
-    // than others (blocks in turn -> so: 2.4 M elements, k = 256 173.7 -> 170.5 us; 0.8 M 65.6 -> 62.6; 1.5 M 113.6 -> 107.8; 2.9 M 215.0 -> 210.7; at most 0.5 M: even)
-    const unsigned blocks = std::min(p.blocks, 8u * (unsigned)num_compute_units());
-    auto launch = [&](auto lanes_) {
+    const unsigned blocks = mat_blocks(p.blocks, lanes);
+    mat_variant(lanes, k, blocks < p.blocks, [&](auto lanes_, auto short_, auto turns) {
         constexpr int L = decltype(lanes_)::value;
-        auto run = [&](auto short_) {
-            constexpr bool SHORT = decltype(short_)::value;
-            if (idx) materialize_vec_kernel<true, L, SHORT><<<blocks, NT, 0, s>>>(p);
-            else materialize_vec_kernel<false, L, SHORT><<<blocks, NT, 0, s>>>(p);
-        };
-        if (k <= MAT_SHORT) run(std::true_type{});
-        else run(std::false_type{});
-    };
-    if (lanes == 16) launch(std::integral_constant<int, 16>{});
-    else if (lanes == 4) launch(std::integral_constant<int, 4>{});
-    else launch(std::integral_constant<int, 1>{});
+        constexpr bool SHORT = decltype(short_)::value, TURNS = decltype(turns)::value;
+        if (idx) materialize_vec_kernel<true, L, SHORT, TURNS><<<blocks, NT, 0, s>>>(p);
+        else materialize_vec_kernel<false, L, SHORT, TURNS><<<blocks, NT, 0, s>>>(p);
+    });
     return check_launch("materialize_vec_kernel");
 }
 
@@ -798,15 +809,10 @@ extern "C" int rdb_materialize_weight_and_bias(float *weight, int64_t n, const f
         };
         const MatVecParams w = params(weight, coef, scale, k, n, seed), b = params(bias->values, bias->coef, bias->scale, bias->k, bias_n, bias->seed);
         const int lanes = mat_lanes(n, k);
-        const unsigned bias_blocks = b.blocks, blocks = bias_blocks + std::min(w.blocks, 8u * (unsigned)num_compute_units());
-        auto launch = [&](auto lanes_) {
-            constexpr int L = decltype(lanes_)::value;
-            if (k <= MAT_SHORT) materialize_vec_pair_kernel<L, true><<<blocks, NT, 0, s>>>(w, b, bias_blocks);
-            else materialize_vec_pair_kernel<L, false><<<blocks, NT, 0, s>>>(w, b, bias_blocks);
-        };
-        if (lanes == 16) launch(std::integral_constant<int, 16>{});
-        else if (lanes == 4) launch(std::integral_constant<int, 4>{});
-        else launch(std::integral_constant<int, 1>{});
+        const unsigned blocks = mat_blocks(w.blocks, lanes);
+        mat_variant(lanes, k, blocks < w.blocks, [&](auto lanes_, auto short_, auto turns) {
+            materialize_vec_pair_kernel<decltype(lanes_)::value, decltype(short_)::value, decltype(turns)::value><<<b.blocks + blocks, NT, 0, s>>>(w, b, b.blocks);
+        });
         return check_launch("materialize_vec_pair_kernel");
     }
     if (n > 0)

@@ -146,3 +146,25 @@ def test_gradient_at_the_edges_of_a_step(hip, n, k):
     want = d.double() @ noise.double()
     # integers throughout and one rounding of a sum of some sqrt(n), 6e-8 of it; the oracle's noise is rounded to fp32, 4.5e-8 a term at most, of either sign
     assert float((hip.materialize_bwd(d, k, 6).double() - want).abs().max()) < 4e-7 * float(n) ** 0.5
+
+
+@pytest.mark.parametrize("n", [524288, 524289, 1200001])
+@pytest.mark.parametrize("k", [5, 48, 70, 2051])
+def test_blocks_of_one_turn_and_of_several(hip, n, k):
+    """One thread an element, on either side of what is resident at once (eight blocks to each of 256 compute units), alone and beside a bias."""
+    import ctypes
+
+    from randumb_amd import _lib
+
+    class PseudoBias(ctypes.Structure):
+        _fields_ = [("coef", ctypes.c_void_p), ("scale", ctypes.c_void_p), ("values", ctypes.c_void_p), ("k", ctypes.c_int64), ("seed", ctypes.c_uint32)]
+
+    g = torch.Generator(device="cuda").manual_seed(k)
+    c, cb = torch.randn(k, generator=g, device="cuda"), torch.randn(30, generator=g, device="cuda")
+    got = hip.materialize_fwd(c, (n,), (1,), 5, None, False)
+    rows = torch.cat([torch.arange(200), torch.arange(n // 2, n // 2 + 200), torch.arange(524188, 524288), torch.arange(n - 200, n)]).cuda()
+    assert rel(got[rows], hip.sq5_fill_2d(n, k, 5)[rows].double() @ c.double()) < 2e-6   # chains of k terms, 2^-24 each
+    w, b = torch.empty(n, device="cuda"), torch.empty(777, device="cuda")
+    pb = PseudoBias(cb.data_ptr(), None, b.data_ptr(), 30, 6)
+    assert _lib.load().rdb_materialize_weight_and_bias(w.data_ptr(), n, c.data_ptr(), k, 5, None, ctypes.byref(pb), 777, torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(w, got) and torch.equal(b, hip.materialize_fwd(cb, (777,), (1,), 6, None, False))

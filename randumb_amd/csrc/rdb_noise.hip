@@ -678,19 +678,20 @@ static void split_plan(int64_t Nw, int64_t k, int64_t *splits, int64_t *span)
 // lanes per element of a tensor of n values by k terms: as many as fill the chip's 8192 wave slots, of 1, 4, 16
 static int mat_lanes(int64_t n, int64_t k) { return k < 8 ? 1 : n <= (1 << 15) ? 16 : n <= (1 << 17) ? 4 : 1; }
 // as many blocks as are resident at once, which take the elements in turns: their coefficients are read once, and no unit is left with a block more
-// than others (blocks in turn -> so: 2.4 M elements, k = 256 173.7 -> 170.5 us; 0.8 M 65.6 -> 62.6; 1.5 M 113.6 -> 107.8; 2.9 M 215.0 -> 210.7; at most 0.5 M: even).  Several lanes to an
-// element: few elements.
-static unsigned mat_blocks(unsigned all, int lanes) { return lanes > 1 ? all : std::min(all, 8u * (unsigned)num_compute_units()); }
+// than others (blocks in turn -> so: 2.4 M elements, k = 256 173.7 -> 170.5 us; 0.8 M 65.6 -> 62.6; 1.5 M 113.6 -> 107.8; 2.9 M 215.0 -> 210.7; at most 0.5 M: even).  Not
+// with few terms, where a turn is short and the loop around it costs more than new blocks do: 0.6 M, k = 9 4.9 us in turn, 5.5 so; 2.4 M, k = 23 25.3, 26.7; 4 M, k = 48 77.9, 82.7, k = 49 79.1, 71.3;
+// 16 M, k = 2 33.5, 29.9, k = 7 59.3, 59.9 (a grid's threads stay below 2^32).  Several lanes to an element: few elements.
+static unsigned mat_blocks(unsigned all, int lanes, int64_t k) { return lanes > 1 || (k <= MAT_SHORT && all < (1u << 24)) ? all : std::min(all, 8u * (unsigned)num_compute_units()); }
 template <class F> static void mat_variant(int lanes, int64_t k, bool turns, F &&f)
 {
-    auto with_terms = [&](auto lanes_, auto turns_) {
-        if (k <= MAT_SHORT) f(lanes_, std::true_type{}, turns_);
-        else f(lanes_, std::false_type{}, turns_);
+    auto with_terms = [&](auto lanes_) {
+        if (k <= MAT_SHORT) f(lanes_, std::true_type{}, std::false_type{});
+        else f(lanes_, std::false_type{}, std::false_type{});
     };
-    if (lanes == 16) with_terms(std::integral_constant<int, 16>{}, std::false_type{});
-    else if (lanes == 4) with_terms(std::integral_constant<int, 4>{}, std::false_type{});
-    else if (turns) with_terms(std::integral_constant<int, 1>{}, std::true_type{});
-    else with_terms(std::integral_constant<int, 1>{}, std::false_type{});
+    if (lanes == 16) with_terms(std::integral_constant<int, 16>{});
+    else if (lanes == 4) with_terms(std::integral_constant<int, 4>{});
+    else if (turns) f(std::integral_constant<int, 1>{}, std::false_type{}, std::true_type{});
+    else with_terms(std::integral_constant<int, 1>{});
 }
 static int launch_materialize_vec(float *out, const void *coef, int coef_dtype, int64_t k, int64_t Nw, int64_t Q, int64_t sP, int64_t sQ, uint32_t seed,
                                   const void *scale_bias, const int64_t *idx, hipStream_t s)
@@ -698,7 +699,7 @@ static int launch_materialize_vec(float *out, const void *coef, int coef_dtype, 
     const int lanes = mat_lanes(Nw, k);
     const MatVecParams p = {out, coef, scale_bias, idx, k, Nw, Q, sP, sQ, coef_dtype, Nw < (1ll << 32) && Q < (1ll << 32), sQ == 1 && (sP == Q || Nw == Q), seed,
                             (unsigned)cdiv(Nw * lanes, NT)};
-    const unsigned blocks = mat_blocks(p.blocks, lanes);
+    const unsigned blocks = mat_blocks(p.blocks, lanes, k);
     mat_variant(lanes, k, blocks < p.blocks, [&](auto lanes_, auto short_, auto turns) {
         constexpr int L = decltype(lanes_)::value;
         constexpr bool SHORT = decltype(short_)::value, TURNS = decltype(turns)::value;
@@ -809,7 +810,7 @@ extern "C" int rdb_materialize_weight_and_bias(float *weight, int64_t n, const f
         };
         const MatVecParams w = params(weight, coef, scale, k, n, seed), b = params(bias->values, bias->coef, bias->scale, bias->k, bias_n, bias->seed);
         const int lanes = mat_lanes(n, k);
-        const unsigned blocks = mat_blocks(w.blocks, lanes);
+        const unsigned blocks = mat_blocks(w.blocks, lanes, k);
         mat_variant(lanes, k, blocks < w.blocks, [&](auto lanes_, auto short_, auto turns) {
             materialize_vec_pair_kernel<decltype(lanes_)::value, decltype(short_)::value, decltype(turns)::value><<<b.blocks + blocks, NT, 0, s>>>(w, b, b.blocks);
         });

@@ -108,7 +108,7 @@ __device__ __forceinline__ void materialize_vec_block(const MatVecParams &p, flo
         if (SHORT || !one_factor) {
             if (live)
                 for (int j = part; j < cnt; j += LANES) {
-                    acc = fmaf(sq5_unit(sq5_tail(first)), cs[j], acc);
+                    acc = fmaf(sq5_unit(sq5_tail_apart(first)), cs[j], acc);
                     first += LANES * SQ5_N1;
                 }
             continue;
@@ -138,7 +138,7 @@ __device__ __forceinline__ void materialize_vec_block(const MatVecParams &p, flo
             if (LANES == 1)
                 for (; j + 4 <= cnt; j += 4) sq5_four_terms(first, sum, *reinterpret_cast<const f32x4 *>(cs + j));
             for (; j < cnt; j += LANES) {
-                sum = fmaf((float)(int32_t)sq5_tail(first), cs[j], sum);
+                sum = fmaf((float)(int32_t)sq5_tail_apart(first), cs[j], sum);
                 first += LANES * SQ5_N1;
             }
             acc = sum * 4.656612873077392578125e-10f;

@@ -524,7 +524,7 @@ int rdb_rms_norm_bwd(void *dx, const void *dy, const void *x, const void *dsum, 
 /* Gradient of a dense embedding table: dweight[v] ([vocab x dim] bf16, overwritten) = sum of the rows of dy ([positions x dim] bf16) with idx[position] == v, in
  * fp32, in a fixed order; indices of idx_bytes 4 or 8; others than 0 .. vocab - 1 count for nothing.  Up to 16384 positions and 2^29 rows, dim a multiple of 8
  * (RDB_E_UNSUPPORTED otherwise); dweight and dy 16-byte aligned.  The first call says for which of these sizes it is the fast way: not for long tables with few positions or
- * columns. */
+ * columns, nor for a few rows with many positions each. */
 int rdb_embedding_bwd_takes(int64_t positions, int64_t vocab, int64_t dim);
 int rdb_embedding_bwd(void *dweight, const void *idx, int idx_bytes, const void *dy, int64_t positions, int64_t vocab, int64_t dim, void *stream);
 

@@ -148,10 +148,13 @@ static bool embedding_fits(int64_t positions, int64_t vocab, int64_t dim)
     return positions > 0 && positions <= EG_POSITIONS && vocab > 0 && vocab <= (1ll << 29) && dim > 0 && dim % 8 == 0 && dim <= (1 << 20);
 }
 
-// Where that is the faster way.  Every block looks through all indices, so a long table costs rounds of blocks, some 12 us each, however few its columns; the stock call costs 25 us with few
-// positions, 55 at 1024, 80 to 110 from there on, and the clearing of the table.  us, this one and the stock one, on either side of each line (256 compute units: a round is 65536 rows):
-//   one round, with few positions and a long or wide table, which is cleared faster than its rows are written one by one: 64 positions, 50304 x 768 22.9, 26.4; 65536 x 768 28.3, 27.7;
-//   50304 x 2048 37.9, 33.1; 512 positions 39.4, 61.4
+// Where that is the faster way.  Every block looks through all indices and writes its rows one by one, so a table costs rounds of blocks, some 12 us each, however few its columns; the stock call
+// adds up positions one after the other, 50 ns each up to 3072 of them, sorts more than that, 55 us, and clears the table, which is faster than rows one by one.  us on the device, this one and the
+// stock one, on either side of each line (256 compute units: a round is 65536 rows):
+//   one round, few positions for the rows: 16384 x 64, 64 positions 8.3, 6.9; 128 8.3, 10.0; 50304 x 256, 256 18.6, 20.2; 128 18.5, 13.6; 65536 x 8, 256 20.5, 16.8; 400 20.6, 24.2; x 768, 128 28.1, 24.1;
+//   256 28.4, 32.3; 32768 x 768, 64 16.6, 14.4; 128 16.8, 18.1
+//   few rows, where a block's eight have most positions: 10 x 384, 1024 positions 33, 48; 10 x 768 60, 48; 30 x 1600, 2048 115, 90; 65 x 1600 29, 88; sorted ones: 65 x 768, 4096 54, 55; 8192 83, 73;
+//   100 x 768, 8192 70, 72; 16384 89, 84; 100 x 1600, 4096 33, 62; 8192 148, 84
 //   rounds against positions: two, x 64 columns: 512 positions 38.1, 32.2; 1024 38.0, 57.8; three: 1024 55.1, 59.8; four: 1024 72.3, 70.6; 2048 73.0, 132
 //   rounds, 4096 positions: four, x 256 74, 95; five 91, 97; seven 112, 100; eight 142, 98; x 768, whose writing takes longer than the indices: eight 187, 198; thirteen 265, 261; a million rows x 8:
 //   246, 99
@@ -159,8 +162,10 @@ extern "C" int rdb_embedding_bwd_takes(int64_t positions, int64_t vocab, int64_t
 {
     if (!embedding_fits(positions, vocab, dim)) return 0;
     const int64_t round = 2 * (int64_t)EG_ROWS * num_compute_units(), rounds = (vocab + round - 1) / round;
-    if (rounds == 1) return positions >= 512 || vocab * dim <= (3 << 24) ? 1 : 0;
-    return rounds <= (dim >= 768 ? 8 : 4) && positions >= 512 * rounds ? 1 : 0;
+    if (rounds > 1) return rounds <= (dim >= 768 ? 8 : 4) && positions >= 512 * rounds ? 1 : 0;
+    if (positions * (dim >= 512 ? 320 : 192) < vocab) return 0;
+    const int64_t pieces = std::min<int64_t>(8, vocab) * ((dim + EG_PIECE - 1) / EG_PIECE);   // of a position in every row of a block, of vocab blocks' worth
+    return positions <= 3072 ? pieces <= vocab : positions * pieces <= 1600 * vocab;
 }
 
 extern "C" int rdb_embedding_bwd(void *dweight, const void *idx, int idx_bytes, const void *dy, int64_t positions, int64_t vocab, int64_t dim, void *stream)

@@ -100,11 +100,13 @@ int rdb_materialize_weight_and_bias(float *weight, int64_t n, const float *coef,
  *   dcoef      [k]
  *   dbias_coef NULL, or [bias_k]: the gradient of a pseudorandom bias's coefficients
  * RDB_E_UNSUPPORTED for empty sizes, matrices of 2^29 elements or more, and while fp32 products are asked for (rdb_set_f32_split); the query then
- * returns 0.  Sums in fixed orders: results are bitwise reproducible run to run. */
+ * returns 0.  Sums in fixed orders: results are bitwise reproducible run to run.  The last call says whether it is the faster way: of dcoef alone only where it saves the
+ * launch that adds up dW's ranges. */
 int64_t rdb_vector_linear_bwd_workspace_bytes(int64_t tokens, int64_t in_f, int64_t out_f, int64_t k, int want_dx, int want_bias);
 int rdb_vector_linear_bwd(float *dx, float *dcoef, float *dbias_coef, const float *dy, int64_t lddy, const float *x, int64_t ldx, const float *W,
                           int64_t tokens, int64_t in_f, int64_t out_f, int64_t k, uint32_t seed, int64_t bias_k, uint32_t bias_seed,
                           void *workspace, int64_t workspace_bytes, void *stream);
+int rdb_vector_linear_bwd_pays(int64_t tokens, int64_t in_f, int64_t out_f, int want_dx, int want_bias);
 
 /* Replaces: op rten::materialize_bwd + materialize_bwd_kernel (R.py:304-359, 383-390).
  * dW is a contiguous tensor of Nw elements (dtype dw_dtype).  dcoef is fp32 and is OVERWRITTEN:

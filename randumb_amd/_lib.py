@@ -35,6 +35,7 @@ EXPORTS = [
     "rdb_materialize_weight_and_bias",
     "rdb_vector_linear_bwd",
     "rdb_vector_linear_bwd_workspace_bytes",
+    "rdb_vector_linear_bwd_pays",
     "rdb_materialize_bwd",
     "rdb_materialize_bwd_workspace_bytes",
     "rdb_scale_bias_bwd",
@@ -182,6 +183,8 @@ def load() -> ctypes.CDLL:
     L.rdb_vector_linear_bwd.restype = ci
     L.rdb_vector_linear_bwd_workspace_bytes.argtypes = [i64, i64, i64, i64, ci, ci]
     L.rdb_vector_linear_bwd_workspace_bytes.restype = i64
+    L.rdb_vector_linear_bwd_pays.argtypes = [i64, i64, i64, ci, ci]
+    L.rdb_vector_linear_bwd_pays.restype = ci
     L.rdb_materialize_fwd.argtypes = [vp, vp, ci, i64, i64, i64, i64, i64, i64, i64, u32, vp, vp]
     L.rdb_materialize_bwd.argtypes = [vp, vp, ci, i64, i64, i64, i64, u32, vp, i64, vp]
     L.rdb_materialize_bwd_workspace_bytes.argtypes = [i64, i64, i64, i64]

@@ -725,6 +725,14 @@ int64_t vector_products_workspace(int64_t tokens, int64_t in_f, int64_t out_f, b
     const int dw = vector_dw_room(tokens, in_f, out_f, want_dx, num_cus);
     return (r > 1 ? r : 0) * up256(tokens * in_f * 4) + (dw > VECTOR_DW_PARTS ? dw + 1 : dw) * up256(out_f * in_f * 4);
 }
+static FgPlan vector_dw_plan(int64_t tokens, int64_t in_f, int64_t out_f, bool dx, int num_cus)
+{
+    return fg_plan(out_f, in_f, tokens, num_cus, vector_dw_room(tokens, in_f, out_f, dx, num_cus), FgGroups<FG_MCONT, FG_MCONT>::four);
+}
+int vector_dw_ranges(int64_t tokens, int64_t in_f, int64_t out_f)
+{
+    return vector_products_ok(tokens, in_f, out_f) ? vector_dw_plan(tokens, in_f, out_f, false, num_compute_units()).ranges : 0;
+}
 int vector_products(float *dx, const float *dy, int64_t lddy, const float *x, int64_t ldx, const float *W, int64_t tokens, int64_t in_f, int64_t out_f,
                     void *workspace, FgSum *dx_sum, VectorDW *dw, hipStream_t s)
 {
@@ -771,7 +779,7 @@ int vector_products(float *dx, const float *dy, int64_t lddy, const float *x, in
         if (int rx = fg_launch<FG_KCONT, FG_MCONT>(qx, num_cus, s, "f32_gemm_kernel (dx = dy . W)")) return rx;
         *dx_sum = fg_sum(dx, 0, dx_part, qx.M * qx.N, dx_stride, px.ranges);
     }
-    const FgPlan pw = fg_plan(qw.M, qw.N, qw.K, num_cus, dw_room, FgGroups<FG_MCONT, FG_MCONT>::four);
+    const FgPlan pw = vector_dw_plan(tokens, in_f, out_f, dx != nullptr, num_cus);
     qw.bm = pw.bm;
     qw.groups = pw.groups;
     ranges(qw, pw.ranges, dw_part, dw_stride);

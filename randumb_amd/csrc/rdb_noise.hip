@@ -1100,6 +1100,17 @@ extern "C" int64_t rdb_vector_linear_bwd_workspace_bytes(int64_t tokens, int64_t
     return vector_bwd_plan(v, tokens, in_f, out_f, k, want_dx != 0, want_bias != 0) ? v.bytes : 0;
 }
 
+// Of dcoef alone: only where the contraction adds up dW's ranges on its way, which saves a launch.  With one range, or more than it adds up, the launches are as many, and its kernel, which could carry more, takes 1 to
+// 3 us longer: on the device, a step, calls of their own and this one: 29 tokens x 8 -> 10, k = 4 14.0, 15.0; 59 x 78 -> 1915, k = 4 26.2, 27.4; 2 x 769 -> 314, k = 14 30.7, 32.4; 13448 x 1031 -> 73, k = 4
+// 88.8, 91.8; two ranges to eight: 333 x 84 -> 23, k = 12 30.0, 21.0; 443 x 42 -> 287, k = 4 24.9, 22.6; 594 x 781 -> 743, k = 3 57.6, 55.2.
+extern "C" int rdb_vector_linear_bwd_pays(int64_t tokens, int64_t in_f, int64_t out_f, int want_dx, int want_bias)
+{
+    VectorBwdPlan v;
+    if (!vector_bwd_plan(v, tokens, in_f, out_f, 1, want_dx != 0, want_bias != 0)) return 0;
+    const int ranges = vector_dw_ranges(tokens, in_f, out_f);
+    return want_dx || want_bias || (ranges > 1 && ranges <= VECTOR_DW_PARTS) ? 1 : 0;
+}
+
 extern "C" int rdb_vector_linear_bwd(float *dx, float *dcoef, float *dbias_coef, const float *dy, int64_t lddy, const float *x, int64_t ldx, const float *W, int64_t tokens,
                                      int64_t in_f, int64_t out_f, int64_t k, uint32_t seed, int64_t bias_k, uint32_t bias_seed, void *workspace, int64_t workspace_bytes,
                                      void *stream)

@@ -64,6 +64,7 @@ struct VectorDW {
 constexpr int VECTOR_DW_PARTS = 8;   // what the contraction with the noise holds on the way
 // rdb_f32.hip
 int64_t vector_products_workspace(int64_t tokens, int64_t in_f, int64_t out_f, bool want_dx);
+int vector_dw_ranges(int64_t tokens, int64_t in_f, int64_t out_f);   // of dW's product without dx beside it; 0: not taken
 int vector_products(float *dx, const float *dy, int64_t lddy, const float *x, int64_t ldx, const float *W, int64_t tokens, int64_t in_f, int64_t out_f,
                     void *workspace, FgSum *dx_sum, VectorDW *dw, hipStream_t s);
 }  // namespace rdb

@@ -794,7 +794,7 @@ class VectorLinear : public Function<VectorLinear> {
         const bool b_coef = bm[0] >= 0 && ctx->needs_input_grad(bias_at), b_scale = bm[0] >= 0 && bm[3] >= 0 && ctx->needs_input_grad(bias_at + 1);
         if (want_c && !want_s && !b_scale && !(b_coef && bm[1] < 0) && dy.scalar_type() == at::kFloat && x0.scalar_type() == at::kFloat && dy.numel() && x0.numel()) {
             const int64_t k = coef.numel(), bk = b_coef ? bm[0] : 0, need = rdb_vector_linear_bwd_workspace_bytes(dy.size(0), l.in_f, l.out_f, k, want_x, bk > 0);
-            if (need > 0) {
+            if (need > 0 && rdb_vector_linear_bwd_pays(dy.size(0), l.in_f, l.out_f, want_x, bk > 0)) {
                 const Tensor x = act(x0.reshape({-1, l.in_f})), ws = bytes(need, dy);
                 const auto f32 = dy.options();
                 if (want_x) dx = at::empty(x0.sizes(), f32);

@@ -38,6 +38,14 @@ def test_a_long_product_of_dw_alone_has_room_for_ranges(tokens, in_f, out_f):
     assert lib.rdb_vector_linear_bwd_workspace_bytes(tokens, in_f, out_f, 8, 0, 0) >= min(lib.rdb_product_f32_workspace_bytes(out_f, in_f, tokens), 28 << 20)
 
 
+@pytest.mark.parametrize("tokens,in_f,out_f,alone", [(29, 8, 10, 0), (2, 769, 314, 0), (59, 78, 1915, 0), (13448, 1031, 73, 0), (8169, 9, 2565, 0), (333, 84, 23, 1), (443, 42, 287, 1), (8192, 768, 3072, 1)])
+def test_where_a_vector_coef_gradient_alone_pays_in_one_call(tokens, in_f, out_f, alone):
+    """Where it saves the launch that adds up dW's ranges; with dx or a bias it saves others."""
+    lib = _lib.load()
+    assert [lib.rdb_vector_linear_bwd_pays(tokens, in_f, out_f, dx, bias) for dx, bias in ((0, 0), (0, 1), (1, 0), (1, 1))] == [alone, 1, 1, 1]
+    assert lib.rdb_vector_linear_bwd_pays(0, in_f, out_f, 1, 1) == 0
+
+
 @pytest.mark.parametrize("dtype", [_lib.RDB_BF16, _lib.RDB_F32])
 def test_nothing_but_what_the_backward_pass_reads(dtype):
     lib, rng = _lib.load(), random.Random(3)

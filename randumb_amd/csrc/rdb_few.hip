@@ -25,6 +25,7 @@
 namespace rdb {
 
 int f32_split_mode();   // rdb_f32.hip
+int num_compute_units();   // rdb_error.hip
 
 constexpr int FEW_ROWS = 64;       // output features of an expanding block: 16 a wave
 constexpr int FEW_COEFS = 16;      // coefficients of a contracting block
@@ -263,7 +264,7 @@ template <typename E, int TT, int WAVES> __device__ __forceinline__ void few_con
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
         const int t = tt * 16 + (tid >> 4);
-        if (t < T && tid < 256) {
+        if (t < T && (WAVES <= 4 || tid < 256)) {
             float *const out = p.part + (((int64_t)ch * p.tiles + tile0 + tt) * p.ranges + range) * p.tile * 16;
             float v = lds[tt * 256 + tid];
 #pragma unroll
@@ -285,7 +286,7 @@ template <typename E, int KS, int TT, bool MANY, int WAVES> __device__ __forcein
     // the wave's rows of C, before anything is waited for
     FewRaw<E> c[KS];
     {
-        const bool ok = wave < 4 && o0 + r < p.out_f;
+        const bool ok = (WAVES <= 4 || wave < 4) && o0 + r < p.out_f;
         const E *const row = static_cast<const E *>(p.coef) + (int64_t)(ok ? o0 + r : 0) * p.k;
 #pragma unroll
         for (int s = 0; s < KS; ++s) c[s] = few_load<E>(row, s * 32 + g * 8, p.k, ok, p.c_vec);
@@ -377,7 +378,7 @@ template <typename E, int KS, int TT, bool MANY, int WAVES> __device__ __forcein
             *reinterpret_cast<uint2 *>(planes + pl * PLANE + (row - pl * T) * LD + p.ranges * FEW_COEFS + (e - row * tail4) * 4) = make_uint2(0u, 0u);
         }
     __syncthreads();
-    if (wave >= 4) return;
+    if (WAVES > 4 && wave >= 4) return;
     f32x4 acc[TT], low[TT];
     auto product = [&](auto any) __attribute__((always_inline)) {
         constexpr bool ANY = decltype(any)::value;
@@ -490,14 +491,16 @@ template <typename E, int TC, int WAVES> __global__ __launch_bounds__(WAVES * 64
 // a chunk of 512 is 16 waves, or 8 where an expanding block is as large (more have no registers for that; k > 256: four).  us per call, four waves -> so: 16 x 4096 -> 11008, k = 256,
 // bf16 11.3 -> 10.7 to 11.2; 64 tokens 18.6 -> 17.3; 8 x 8192 -> 8192, k = 512 21.9 -> 19.9; in one launch: 1 x 4096 -> 4096, k = 16, fp32 8.9 -> 8.1; 4 x 2000 -> 5000, k = 100 9.5 -> 8.7;
 // 16 x 4096 -> 4096, k = 128 11.1 -> 10.6.  (Chunks of 1024 and 2048 in 16 waves, half and a quarter of the partial sums: 11.8 and 15.1 for the first.  Expanding blocks of eight waves in
-// a launch of their own: 64 tokens 20.7.)  The number depends on the layer alone, so that the same sums come out in one launch and in two.
+// a launch of their own: 64 tokens 20.7.)  In one launch four again where the blocks are more than the compute units, of which eight waves have one each: 1 x 7728 -> 273, k = 255, 261 blocks, fp32 12.5,
+// eight 15.2; 324 x 1449 -> 373, k = 67, bf16 17.1, 17.9; and where a chunk of 256 for k > 128 is one step a wave, which the sums of eight cost more than, up to 10 tokens: 3 x 1425 -> 4496, k = 187, fp32 10.6, 11.2; 2 x
+// 1390 -> 4751, k = 132, bf16 9.2, 9.6; but 15 x 1202 -> 460, k = 208 11.8, 10.4.  The number depends on the layer and its tokens alone, so that the same sums come out in one launch and in two.
 // te: tiles of an expanding block.  Finer is sooner ready while the blocks run side by side, two (of k > 128: one) to a compute unit: 64 x
 // 768 -> 3072, k = 64: 8.2 us, two tiles 9.1; 80 x 8192 -> 8192, k = 64, 640 blocks of one tile: 18.7, two tiles 15.1.
 // sum: beyond 200 KB of partial sums for a block they are added up once, by a launch of its own, and not by every expanding block
 // (48 to a block, 32 tokens x 4096 -> 11008, k = 256: 15.6 -> 14.9 us; 16 tokens, 131 KB: 11.5, and 12.7 with it).
 // one: a single launch where the expanding blocks are few and the partial sums of each small; tags and reads that go around L2 cost many
 // blocks more than a launch does (16 x 4096 -> 11008, k = 256: two launches 11.5, one 13.5), but a program's host takes 9.0 to 11.7 us (by
-// the box and by what the program does between calls) to issue two, and those calls then take that.  us of a call in one launch, which
+// the machine and by what the program does between calls) to issue two, and those calls then take that.  us of a call in one launch, which
 // the host does not hold up: (two launches wait for the host, 10.0 and more) 1 x 2048 -> 11008, k = 64, 172 blocks, 32 tags: 8.7; 8 tokens, 16 KB a block: 9.1, but 1 x 4096 ->
 // 11008, k = 256, 128 tags 10.4, 2 x 4096 -> 16000, k = 128, 250 blocks 10.5; earlier, with four waves: 5 x 1001 -> 999, k = 99: 7.8; 48 x 768 -> 768, k = 64: 8.3; 100 x 264 -> 352, k = 64: 8.7; 32 x 1024 -> 2048,
 // k = 128, 64 blocks of 64 KB: 9.2; 4 x 2048 -> 10000, k = 32, 157 blocks: 9.0; 64 x 768 -> 2048, k = 64, 128 blocks: 9.9.  At the line the
@@ -533,7 +536,8 @@ static FewPlan few_plan(const rdb_linear_desc *d)
     const int64_t block_bytes = f.chunks * per_chunk * std::min(f.te, f.tiles);   // what an expanding block reads
     f.one = !f.sum && ((f.e_blocks <= 64 && block_bytes <= 100 * 1024) || (f.e_blocks <= 160 && block_bytes <= 32 * 1024) ||
                        (f.e_blocks <= 192 && block_bytes <= 16 * 1024 && f.c_blocks <= 32));
-    f.waves = (int)std::min<int64_t>(f.one ? (d->k <= 256 ? 8 : 4) : 16, chunk / 32);
+    const bool four = d->k > 256 || f.c_blocks + f.e_blocks > num_compute_units() || (d->k > 128 && chunk <= 256 && f.tile <= 10);
+    f.waves = (int)std::min<int64_t>(f.one ? (four ? 4 : 8) : 16, chunk / 32);
     f.wave_values = (int)chunk / f.waves;
     return f;
 }

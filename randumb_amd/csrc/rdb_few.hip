@@ -501,11 +501,13 @@ template <typename E, int TC, int WAVES> __global__ __launch_bounds__(WAVES * 64
 // one: a single launch where the expanding blocks are few and the partial sums of each small; tags and reads that go around L2 cost many
 // blocks more than a launch does (16 x 4096 -> 11008, k = 256: two launches 11.5, one 13.5), but a program's host takes 9.0 to 11.7 us (by
 // the machine and by what the program does between calls) to issue two, and those calls then take that.  us of a call in one launch, which
-// the host does not hold up: (two launches wait for the host, 10.0 and more) 1 x 2048 -> 11008, k = 64, 172 blocks, 32 tags: 8.7; 8 tokens, 16 KB a block: 9.1, but 1 x 4096 ->
-// 11008, k = 256, 128 tags 10.4, 2 x 4096 -> 16000, k = 128, 250 blocks 10.5; earlier, with four waves: 5 x 1001 -> 999, k = 99: 7.8; 48 x 768 -> 768, k = 64: 8.3; 100 x 264 -> 352, k = 64: 8.7; 32 x 1024 -> 2048,
+// the host does not hold up: 5 x 1001 -> 999, k = 99: 7.8; 48 x 768 -> 768, k = 64: 8.3; 100 x 264 -> 352, k = 64: 8.7; 32 x 1024 -> 2048,
 // k = 128, 64 blocks of 64 KB: 9.2; 4 x 2048 -> 10000, k = 32, 157 blocks: 9.0; 64 x 768 -> 2048, k = 64, 128 blocks: 9.9.  At the line the
 // two are about even, whichever the host: 256 x 512 -> 640, k = 128, 160 blocks of 32 KB and 256 tags: 10.7 in bf16 and 11.6 in fp32, two launches
 // 9.3 and 9.7 on the fastest host, 11.7 and 11.5 in a program; 224 x 512 -> 640, k = 96, 140 blocks, 168 tags, bf16: 12.2, and 9.5 or 11.3.
+// More blocks only for sizes that are other kernels' in two launches (few_one_or_none), up to 192 of 16 KB and 32 tags, on the device: 2 x 395 -> 11221, k = 125 16.0, 8.6; 48 x 237 -> 3841, k = 116 15.5, 10.6;
+// 107 x 226 -> 1452, k = 21 13.5, 10.2, but 97 x 91 -> 1616, k = 18 9.8, 10.6.  Others of that many, two launches and one: 1 x 267 -> 10914, k = 48 7.4, 9.6; 51 x 327 -> 2944, k = 32 8.9, 10.9; 20 x 1840 ->
+// 5285, k = 8 9.1, 11.2; 6 x 2028 -> 10953, k = 7 8.8, 10.1.
 struct FewPlan {
     int wave_values, waves, chunks, ranges;   // waves: of a contracting block, and of both kinds where they are one launch
     int tile, tiles, tc, te;
@@ -513,6 +515,11 @@ struct FewPlan {
     bool sum, one;
     int64_t part_bytes;
 };
+// short contractions in bf16, which are other kernels' in two launches (few_pays)
+static bool few_one_or_none(const rdb_linear_desc *d)
+{
+    return d->act_dtype == RDB_BF16 && d->in_f < 512 && (d->k > 64 || (d->tokens > 96 && d->in_f > 128));
+}
 static FewPlan few_plan(const rdb_linear_desc *d)
 {
     FewPlan f;
@@ -535,7 +542,7 @@ static FewPlan few_plan(const rdb_linear_desc *d)
     f.e_blocks = (int)(rows * cdiv(f.tiles, f.te));
     const int64_t block_bytes = f.chunks * per_chunk * std::min(f.te, f.tiles);   // what an expanding block reads
     f.one = !f.sum && ((f.e_blocks <= 64 && block_bytes <= 100 * 1024) || (f.e_blocks <= 160 && block_bytes <= 32 * 1024) ||
-                       (f.e_blocks <= 192 && block_bytes <= 16 * 1024 && f.c_blocks <= 32));
+                       (few_one_or_none(d) && f.e_blocks <= 192 && block_bytes <= 16 * 1024 && f.c_blocks <= 32));
     const bool four = d->k > 256 || f.c_blocks + f.e_blocks > num_compute_units() || (d->k > 128 && chunk <= 256 && f.tile <= 10);
     f.waves = (int)std::min<int64_t>(f.one ? (four ? 4 : 8) : 16, chunk / 32);
     f.wave_values = (int)chunk / f.waves;

@@ -94,8 +94,8 @@ int rdb_materialize_weight_and_bias(float *weight, int64_t n, const float *coef,
                                     const rdb_pseudo_bias *bias, int64_t bias_n, void *stream);
 
 /* Backward pass of a vector-coef layer in fp32, y = x . W^T + b with W [out_f x in_f] and b formed by rdb_materialize_fwd: what two calls of
- * rdb_product_f32 (dx = dy . W, dW = dy^T . x), rdb_materialize_bwd on dW and rdb_bias_bwd give, in three launches (four where the
- * products cannot share one); dW is not kept.
+ * rdb_product_f32 (dx = dy . W, dW = dy^T . x), rdb_materialize_bwd on dW and rdb_bias_bwd give, in three launches (one more where the
+ * products cannot share one, and where dW's product is in more ranges than the contraction adds up); dW is not kept.
  *   dx         NULL, or [tokens x in_f], contiguous (W is read then)
  *   dcoef      [k]
  *   dbias_coef NULL, or [bias_k]: the gradient of a pseudorandom bias's coefficients

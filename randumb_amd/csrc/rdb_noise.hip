@@ -1070,7 +1070,7 @@ extern "C" int rdb_bias_bwd(float *dcoef, float *ds, const void *dy, int dtype, 
 // As calls of their own: dx and dW, a product and a sum of its ranges each, dW's contraction with the noise and the sum of its partial rows, the
 // column sums of dy and the bias's contraction, eight launches of which six are 5 to 8 us and a gap behind each.  Here three: the two products side by
 // side, the contraction, which adds dW's ranges up on the way and has dx's sums and the column sums beside it (it is the vector ALU's, they are the memory's), and the
-// small ends together.  Step of 1024 tokens x 768 -> 3072, k = 256: 481 -> 466 us (1.3 % of it for the bias's values formed beside W's in the forward pass); 1024 x 512 ->
+// small ends together; more than VECTOR_DW_PARTS ranges of dW, many tokens of a small layer, are added up by a fourth.  Step of 1024 tokens x 768 -> 3072, k = 256: 481 -> 466 us (1.3 % of it for the bias's values formed beside W's in the forward pass); 1024 x 512 ->
 // 1024, k = 200: 131 -> 118; steps that wait for the host, 2048 x 256 -> 512, k = 100: 100 -> 81; 32 x 64 -> 64, k = 16: 90 -> 79.
 namespace rdb {
 

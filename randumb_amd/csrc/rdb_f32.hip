@@ -709,12 +709,15 @@ static bool vector_products_ok(int64_t tokens, int64_t in_f, int64_t out_f)
 // 147, 130, 131; 2048 x 1024 -> 1024, k = 256 256, 245, 245, 244; 1024 x 768 -> 3072, k = 256, kept up for a second: 464, 475, 475, 477.
 // Many tokens of a small layer are more ranges than the contraction holds on the way (VECTOR_DW_PARTS): they and dx's are added up by a launch of their own then.  Eight at most
 // and so, us: 30138 x 111 -> 331, k = 111 217, 131 (eight launches 145); 13811 x 135 -> 211, k = 52 96, 80 (85); 9080 x 280 -> 560, k = 18 130, 109 (118).
-// Without dx beside it, whose tiles fill its last round, a long product of dW (2048 tokens and more) loses more to that round: 32 MB there.  No dx, 16 and 32 MB: 8192 x 768 -> 3072, k = 8
-// 539, 442 (469 as calls of their own); 19876 x 1288 -> 680, k = 4 539, 486 (501); 16384 x 1024 -> 1024, k = 8 384, 386; 1024 x 768 -> 3072, k = 256 447, 452; with dx 16384 x 1024 ->
-// 1024 514, 551, 32768 x 512 -> 512, k = 8 313, 334.
+// Without dx beside it, whose tiles fill its last round, a product of dW that is not short (1280 tokens and more) loses more to that round: 32 MB there.  No dx, 16 and 32 MB: 8192 x 768 -> 3072, k = 8
+// 539, 442 (469 as calls of their own); 19876 x 1288 -> 680, k = 4 539, 486 (501); 16384 x 1024 -> 1024, k = 8 384, 386; 1722 x 1388 -> 1566, k = 8 217, 191 (199); 1024 x 768 -> 3072, k = 256 447, 452; with dx
+// 16384 x 1024 -> 1024 514, 551, 32768 x 512 -> 512, k = 8 313, 334.
+// With dx one range of dW is tiles that run as long as the whole launch, each beside others on its unit, where they are less than two to three units: two ranges there.  Steps with one and two: 8192 x 1388 -> 1566, k = 8
+// 993, 813 (892 as calls of their own); 8192 x 1771 -> 1463 1042, 956 (962); 4096 x 768 -> 3072, k = 256 778, 726 (831); 1400 tokens of it 527, 531, 1250 493, 501; 8192 x 2000 -> 2000, 256 tiles, one range: 1199 (1211).
 static int vector_dw_room(int64_t tokens, int64_t in_f, int64_t out_f, bool dx, int num_cus)
 {
-    const int64_t most = std::max<int64_t>(1, (dx || tokens < 2048 ? 16 << 20 : 32 << 20) / (out_f * in_f * 4));
+    const bool few_tiles = 3 * cdiv(out_f, 128) * cdiv(in_f, 128) < 2 * num_cus;
+    const int64_t most = std::max<int64_t>(few_tiles && tokens >= 1280 ? 2 : 1, (dx || tokens < 1280 ? 16 << 20 : 32 << 20) / (out_f * in_f * 4));
     return (int)std::min<int64_t>(product_room(out_f, in_f, tokens, num_cus), most);
 }
 // scratch: dx's partial matrices and dW's (or dW); 0: not taken

@@ -130,3 +130,9 @@ def test_backward_pass_in_one_call(tokens, in_f, out_f, k, bias_k):
         if bias_k:
             assert _rel(db, (dy.double().sum(0) @ hip.sq5_fill_2d(out_f, bias_k, 4).double()).cpu()) < 3e-6
         assert call(need - 1) < 0
+
+
+# few tiles of a large dW: one range and two beside dx, one and three alone
+@pytest.mark.parametrize("tokens,in_f,out_f,k", [(1279, 1388, 1566, 6), (1280, 1388, 1566, 6)])
+def test_backward_pass_of_a_dw_of_few_tiles(tokens, in_f, out_f, k):
+    test_backward_pass_in_one_call(tokens, in_f, out_f, k, 0)

@@ -38,6 +38,13 @@ def test_a_long_product_of_dw_alone_has_room_for_ranges(tokens, in_f, out_f):
     assert lib.rdb_vector_linear_bwd_workspace_bytes(tokens, in_f, out_f, 8, 0, 0) >= min(lib.rdb_product_f32_workspace_bytes(out_f, in_f, tokens), 28 << 20)
 
 
+@pytest.mark.parametrize("tokens,in_f,out_f,dx,ranges", [(1722, 1388, 1566, 0, 3), (8192, 1388, 1566, 1, 2), (8192, 1771, 1463, 1, 2), (1400, 768, 3072, 1, 2)])
+def test_a_dw_of_few_tiles_has_room_for_ranges(tokens, in_f, out_f, dx, ranges):
+    """Fewer tiles than two to three compute units: in one range they are the last to be done, with dx beside them too."""
+    lib = _lib.load()
+    assert lib.rdb_vector_linear_bwd_workspace_bytes(tokens, in_f, out_f, 8, dx, 0) >= ranges * in_f * out_f * 4
+
+
 @pytest.mark.parametrize("tokens,in_f,out_f,alone", [(29, 8, 10, 0), (2, 769, 314, 0), (59, 78, 1915, 0), (13448, 1031, 73, 0), (8169, 9, 2565, 0), (333, 84, 23, 1), (443, 42, 287, 1), (8192, 768, 3072, 1)])
 def test_where_a_vector_coef_gradient_alone_pays_in_one_call(tokens, in_f, out_f, alone):
     """Where it saves the launch that adds up dW's ranges; with dx or a bias it saves others."""

@@ -491,9 +491,11 @@ template <typename E, int TC, int WAVES> __global__ __launch_bounds__(WAVES * 64
 // a chunk of 512 is 16 waves, or 8 where an expanding block is as large (more have no registers for that; k > 256: four).  us per call, four waves -> so: 16 x 4096 -> 11008, k = 256,
 // bf16 11.3 -> 10.7 to 11.2; 64 tokens 18.6 -> 17.3; 8 x 8192 -> 8192, k = 512 21.9 -> 19.9; in one launch: 1 x 4096 -> 4096, k = 16, fp32 8.9 -> 8.1; 4 x 2000 -> 5000, k = 100 9.5 -> 8.7;
 // 16 x 4096 -> 4096, k = 128 11.1 -> 10.6.  (Chunks of 1024 and 2048 in 16 waves, half and a quarter of the partial sums: 11.8 and 15.1 for the first.  Expanding blocks of eight waves in
-// a launch of their own: 64 tokens 20.7.)  In one launch four again where the blocks are more than the compute units, of which eight waves have one each: 1 x 7728 -> 273, k = 255, 261 blocks, fp32 12.5,
-// eight 15.2; 324 x 1449 -> 373, k = 67, bf16 17.1, 17.9; and where a chunk of 256 for k > 128 is one step a wave, which the sums of eight cost more than, up to 10 tokens: 3 x 1425 -> 4496, k = 187, fp32 10.6, 11.2; 2 x
-// 1390 -> 4751, k = 132, bf16 9.2, 9.6; but 15 x 1202 -> 460, k = 208 11.8, 10.4.  The number depends on the layer and its tokens alone, so that the same sums come out in one launch and in two.
+// a launch of their own: 64 tokens 20.7.)  In one launch four again where eight cost more.  Of eight waves a unit has one block: contracting
+// blocks of fp32 that are more than the units, 460 x 1862 -> 164, k = 40, 360 blocks 16.8, four 15.4; 511 x 5005 -> 267, k = 47 24.9, 22.7 (bf16 either way: 106 x 1923 -> 371, k = 136 16.7, 15.9; 242 x 8261 -> 92, k = 27 18.8, 20.9; fewer
+// blocks: 235 x 3014 -> 491, k = 57, 192 and 120 14.8, 17.6), and of one tile of tokens and k > 128 all blocks, whose sums are a wait: 1 x 7728 -> 273, k = 255, 261 of them, 15.2, 12.5; 4 x 1833 -> 9483, k = 213 14.0, 12.2.  A chunk of 256 for
+// k > 128, one step a wave, which the sums of eight cost more than up to 10 tokens: 3 x 1425 -> 4496, k = 187, fp32 11.2, 10.6; 2 x 1390 -> 4751, k = 132, bf16 9.6, 9.2; but 15 x 1202 -> 460, k = 208 10.4, 11.8.
+// The number depends on the layer and its tokens alone, so that the same sums come out in one launch and in two.
 // te: tiles of an expanding block.  Finer is sooner ready while the blocks run side by side, two (of k > 128: one) to a compute unit: 64 x
 // 768 -> 3072, k = 64: 8.2 us, two tiles 9.1; 80 x 8192 -> 8192, k = 64, 640 blocks of one tile: 18.7, two tiles 15.1.
 // sum: beyond 200 KB of partial sums for a block they are added up once, by a launch of its own, and not by every expanding block
@@ -543,7 +545,8 @@ static FewPlan few_plan(const rdb_linear_desc *d)
     const int64_t block_bytes = f.chunks * per_chunk * std::min(f.te, f.tiles);   // what an expanding block reads
     f.one = !f.sum && ((f.e_blocks <= 64 && block_bytes <= 100 * 1024) || (f.e_blocks <= 160 && block_bytes <= 32 * 1024) ||
                        (few_one_or_none(d) && f.e_blocks <= 192 && block_bytes <= 16 * 1024 && f.c_blocks <= 32));
-    const bool four = d->k > 256 || f.c_blocks + f.e_blocks > num_compute_units() || (d->k > 128 && chunk <= 256 && f.tile <= 10);
+    const bool four = d->k > 256 || (f.tc == 1 ? d->k > 128 && (f.c_blocks + f.e_blocks > num_compute_units() || (chunk <= 256 && f.tile <= 10))
+                                               : d->act_dtype == RDB_F32 && f.c_blocks > num_compute_units());
     f.waves = (int)std::min<int64_t>(f.one ? (four ? 4 : 8) : 16, chunk / 32);
     f.wave_values = (int)chunk / f.waves;
     return f;

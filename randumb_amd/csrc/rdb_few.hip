@@ -507,9 +507,9 @@ template <typename E, int TC, int WAVES> __global__ __launch_bounds__(WAVES * 64
 // k = 128, 64 blocks of 64 KB: 9.2; 4 x 2048 -> 10000, k = 32, 157 blocks: 9.0; 64 x 768 -> 2048, k = 64, 128 blocks: 9.9.  At the line the
 // two are about even, whichever the host: 256 x 512 -> 640, k = 128, 160 blocks of 32 KB and 256 tags: 10.7 in bf16 and 11.6 in fp32, two launches
 // 9.3 and 9.7 on the fastest host, 11.7 and 11.5 in a program; 224 x 512 -> 640, k = 96, 140 blocks, 168 tags, bf16: 12.2, and 9.5 or 11.3.
-// More blocks only for sizes that are other kernels' in two launches (few_one_or_none), up to 192 of 16 KB and 32 tags, on the device: 2 x 395 -> 11221, k = 125 16.0, 8.6; 48 x 237 -> 3841, k = 116 15.5, 10.6;
-// 107 x 226 -> 1452, k = 21 13.5, 10.2, but 97 x 91 -> 1616, k = 18 9.8, 10.6.  Others of that many, two launches and one: 1 x 267 -> 10914, k = 48 7.4, 9.6; 51 x 327 -> 2944, k = 32 8.9, 10.9; 20 x 1840 ->
-// 5285, k = 8 9.1, 11.2; 6 x 2028 -> 10953, k = 7 8.8, 10.1.
+// More blocks, up to 192 of 16 KB and 32 tags: of one tile of tokens, where two launches wait for the host and one is mostly sooner than that (on the device, two and one, and two called in a loop: 8 x 515 -> 10437, k = 14 8.0,
+// 9.0, 10.4; 4 x 448 -> 10988, k = 5 7.9, 8.7, 9.7; 1 x 267 -> 10914, k = 48 7.4, 9.6, 9.8); of several only for sizes that are other kernels' in two launches (few_one_or_none): 48 x 237 -> 3841, k = 116 15.5, 10.6; 107 x 226 -> 1452,
+// k = 21 13.5, 10.2, but 97 x 91 -> 1616, k = 18 9.8, 10.6; others: 51 x 327 -> 2944, k = 32 8.9, 10.9; 20 x 1840 -> 5285, k = 8 9.1, 11.2.
 struct FewPlan {
     int wave_values, waves, chunks, ranges;   // waves: of a contracting block, and of both kinds where they are one launch
     int tile, tiles, tc, te;
@@ -544,7 +544,7 @@ static FewPlan few_plan(const rdb_linear_desc *d)
     f.e_blocks = (int)(rows * cdiv(f.tiles, f.te));
     const int64_t block_bytes = f.chunks * per_chunk * std::min(f.te, f.tiles);   // what an expanding block reads
     f.one = !f.sum && ((f.e_blocks <= 64 && block_bytes <= 100 * 1024) || (f.e_blocks <= 160 && block_bytes <= 32 * 1024) ||
-                       (few_one_or_none(d) && f.e_blocks <= 192 && block_bytes <= 16 * 1024 && f.c_blocks <= 32));
+                       ((f.tc == 1 || few_one_or_none(d)) && f.e_blocks <= 192 && block_bytes <= 16 * 1024 && f.c_blocks <= 32));
     const bool four = d->k > 256 || (f.tc == 1 ? d->k > 128 && (f.c_blocks + f.e_blocks > num_compute_units() || (chunk <= 256 && f.tile <= 10))
                                                : d->act_dtype == RDB_F32 && f.c_blocks > num_compute_units());
     f.waves = (int)std::min<int64_t>(f.one ? (four ? 4 : 8) : 16, chunk / 32);

@@ -493,8 +493,9 @@ template <typename E, int TC, int WAVES> __global__ __launch_bounds__(WAVES * 64
 // 16 x 4096 -> 4096, k = 128 11.1 -> 10.6.  (Chunks of 1024 and 2048 in 16 waves, half and a quarter of the partial sums: 11.8 and 15.1 for the first.  Expanding blocks of eight waves in
 // a launch of their own: 64 tokens 20.7.)  In one launch four again where eight cost more.  Of eight waves a unit has one block: contracting
 // blocks of fp32 that are more than the units, 460 x 1862 -> 164, k = 40, 360 blocks 16.8, four 15.4; 511 x 5005 -> 267, k = 47 24.9, 22.7 (bf16 either way: 106 x 1923 -> 371, k = 136 16.7, 15.9; 242 x 8261 -> 92, k = 27 18.8, 20.9; fewer
-// blocks: 235 x 3014 -> 491, k = 57, 192 and 120 14.8, 17.6), and of one tile of tokens and k > 128 all blocks, whose sums are a wait: 1 x 7728 -> 273, k = 255, 261 of them, 15.2, 12.5; 4 x 1833 -> 9483, k = 213 14.0, 12.2.  A chunk of 256 for
-// k > 128, one step a wave, which the sums of eight cost more than up to 10 tokens: 3 x 1425 -> 4496, k = 187, fp32 11.2, 10.6; 2 x 1390 -> 4751, k = 132, bf16 9.6, 9.2; but 15 x 1202 -> 460, k = 208 10.4, 11.8.
+// blocks: 235 x 3014 -> 491, k = 57, 192 and 120 14.8, 17.6), and, of one tile of tokens, k > 128 that is no multiple of 8, whose rows of C are read a value at a time, with more blocks in all than
+// units, 1 x 7728 -> 273, k = 255, 261 of them, 15.2, 12.5; 4 x 1833 -> 9483, k = 213 14.0, 12.2 (k = 192, 2 x 5225 -> 7979 13.2, 14.8), or chunks of 256, one step a wave, up to 8 tokens: 3 x 1425 -> 4496, k = 187, fp32 11.2, 10.6; 74
+// and 87 sizes, bf16 and fp32, 0.98 and 0.965 times eight's, but 1.03 and 1.055 where k is a multiple of 8 (5 x 1775 -> 6639, k = 176, bf16 10.2, 11.0), and 15 x 1202 -> 460, k = 208 10.4, 11.8.
 // The number depends on the layer and its tokens alone, so that the same sums come out in one launch and in two.
 // te: tiles of an expanding block.  Finer is sooner ready while the blocks run side by side, two (of k > 128: one) to a compute unit: 64 x
 // 768 -> 3072, k = 64: 8.2 us, two tiles 9.1; 80 x 8192 -> 8192, k = 64, 640 blocks of one tile: 18.7, two tiles 15.1.
@@ -545,7 +546,7 @@ static FewPlan few_plan(const rdb_linear_desc *d)
     const int64_t block_bytes = f.chunks * per_chunk * std::min(f.te, f.tiles);   // what an expanding block reads
     f.one = !f.sum && ((f.e_blocks <= 64 && block_bytes <= 100 * 1024) || (f.e_blocks <= 160 && block_bytes <= 32 * 1024) ||
                        ((f.tc == 1 || few_one_or_none(d)) && f.e_blocks <= 192 && block_bytes <= 16 * 1024 && f.c_blocks <= 32));
-    const bool four = d->k > 256 || (f.tc == 1 ? d->k > 128 && (f.c_blocks + f.e_blocks > num_compute_units() || (chunk <= 256 && f.tile <= 10))
+    const bool four = d->k > 256 || (f.tc == 1 ? d->k > 128 && d->k % 8 && (f.c_blocks + f.e_blocks > num_compute_units() || (chunk <= 256 && f.tile <= 8))
                                                : d->act_dtype == RDB_F32 && f.c_blocks > num_compute_units());
     f.waves = (int)std::min<int64_t>(f.one ? (four ? 4 : 8) : 16, chunk / 32);
     f.wave_values = (int)chunk / f.waves;

@@ -54,7 +54,7 @@ def test_against_float64(T, in_f, out_f, k, dtype):
     assert torch.equal(out[:, :out_f], y) and bool((out[:, out_f:] == 7.0).all())
 
 
-# four waves of a block and eight, in one launch: 8 tokens and 9, chunks of 256 and 512, k = 128 and 129; as many blocks as compute units and one more
+# four waves of a block and eight, in one launch: 8 tokens and 9, chunks of 256 and 512, k below 128 and above, odd and a multiple of 8; as many blocks as compute units and one more
 @pytest.mark.parametrize("T,in_f,out_f,k", [(8, 1030, 130, 129), (8, 1030, 130, 136), (9, 1030, 130, 129), (8, 2048, 64, 255), (8, 2049, 64, 255), (8, 1030, 130, 127), (1, 8000, 64, 255), (1, 7680, 1024, 254), (1, 7680, 1025, 254), (200, 8192, 64, 32), (200, 8192, 64, 48),
                                             (2, 300, 10304, 100), (16, 200, 10304, 30), (51, 327, 2944, 32), (100, 200, 1500, 20), (100, 120, 1500, 20)])   # more than 160 expanding blocks
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
